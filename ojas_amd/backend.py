@@ -19,6 +19,11 @@ from typing import Optional, Sequence, Tuple
 import numpy as np
 
 from . import shapes
+try:
+    from . import _native
+except ImportError as _e:
+    raise ImportError("ojas_amd/_native.so is not built; run __graft_entry__.build()") from _e
+from ._native import DeviceTensor  # a contiguous device tensor (host/py_native.cpp)
 
 LIB_PATH = Path(__file__).resolve().parent / "libojas_mi355x.so"
 
@@ -83,40 +88,6 @@ def load_library() -> C.CDLL:
     return lib
 
 
-class DeviceTensor:
-    """A contiguous device tensor: pointer, shape, dtype. Frees itself on drop
-    (the role of `Arc<dyn DeviceBuffer>` + `Reservation`, tensor.rs:146-163)."""
-
-    def __init__(self, backend: "MiBackend", ptr: int, shape: Tuple[int, ...], dtype: int, owns: bool = True):
-        self.backend, self.ptr, self.shape, self.dtype, self._owns = backend, ptr, tuple(shape), dtype, owns
-        # The storage compute tag of an f32 tensor (tensor.rs COMPUTE_BF16): True when its values are
-        # known to be bf16-exact, so a second rounding would only clone. Set by `Autocast`.
-        self.compute_bf16 = False
-
-    @property
-    def numel(self) -> int:
-        return int(np.prod(self.shape)) if self.shape else 1
-
-    @property
-    def nbytes(self) -> int:
-        return self.numel * _SIZE_OF[self.dtype]
-
-    def reshape(self, *shape) -> "DeviceTensor":
-        """Zero-copy view (tensor.rs:1555-1605); the view does not own the memory."""
-        shape = tuple(shape[0]) if len(shape) == 1 and isinstance(shape[0], (tuple, list)) else tuple(shape)
-        if int(np.prod(shape)) != self.numel:
-            raise OjasError(SHAPE, f"reshape {self.shape} -> {shape}")
-        view = DeviceTensor(self.backend, self.ptr, shape, self.dtype, owns=False)
-        view._base = self
-        view.compute_bf16 = self.compute_bf16
-        return view
-
-    def __del__(self):
-        if getattr(self, "_owns", False) and self.ptr and self.backend is not None and self.backend._ctx:
-            self.backend._lib.omx_free(self.backend._ctx, C.c_void_p(self.ptr))
-            self.ptr = 0
-
-
 class MiBackend:
     """`impl Backend for MiBackend`: BackendId::Hip, Numerics::Fast, bf16 operands accepted."""
 
@@ -126,14 +97,17 @@ class MiBackend:
 
     def __init__(self, device: int = 0, budget_bytes: int = 0):
         self._lib = load_library()
+        _native.load(str(LIB_PATH), OjasError)
         ctx = C.c_void_p()
         rc = self._lib.omx_open(C.c_int32(device), C.c_uint64(budget_bytes), C.byref(ctx))
         self._ctx = ctx if rc == OK else None
+        self._context = _native.Context(ctx.value or 0)
         if rc != OK:
             raise OjasError(rc, "omx_open failed (no gfx950 device or runtime error)")
 
     def close(self):
         if self._ctx:
+            self._context.close()  # tensors still alive no longer free themselves: the context does
             self._lib.omx_close(self._ctx)
             self._ctx = None
 
@@ -158,15 +132,11 @@ class MiBackend:
                 "pooled": int(self._lib.omx_budget_pooled(self._ctx))}
 
     def empty(self, shape, dtype: int = F32) -> DeviceTensor:
-        shape = tuple(int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,)))
-        n = int(np.prod(shape)) if shape else 1
-        ptr = C.c_void_p()
-        self._check(self._lib.omx_alloc(self._ctx, C.c_uint64(max(n, 1) * _SIZE_OF[dtype]), C.byref(ptr)))
-        return DeviceTensor(self, ptr.value, shape, dtype)
+        return _native.empty(self, self._context, shape, dtype)
 
     def zeros(self, shape, dtype: int = F32) -> DeviceTensor:
         t = self.empty(shape, dtype)
-        self._check(self._lib.omx_fill_zero(self._ctx, C.c_void_p(t.ptr), C.c_uint64(t.nbytes)))
+        _native.omx_fill_zero(self._context, t, t.nbytes)
         return t
 
     def upload(self, host: np.ndarray, dtype: Optional[int] = None) -> DeviceTensor:
@@ -185,8 +155,7 @@ class MiBackend:
             raise OjasError(DTYPE, f"upload of {host.dtype}")
         t = self.empty(host.shape, src_dtype)
         if host.size:
-            self._check(self._lib.omx_upload(self._ctx, C.c_void_p(t.ptr), C.c_uint64(0),
-                                             host.ctypes.data_as(C.c_void_p), C.c_uint64(host.nbytes)))
+            _native.omx_upload(self._context, t, 0, host.ctypes.data, host.nbytes)
         if dtype is not None and dtype != src_dtype:
             if src_dtype == F32 and dtype == BF16:
                 return self.to_bf16(t)
@@ -196,8 +165,7 @@ class MiBackend:
     def download(self, t: DeviceTensor) -> np.ndarray:
         """BackendCore::download (backend.rs:938-961): syncs, reports deferred faults."""
         out = np.empty(t.shape, dtype=_NP_OF[t.dtype])
-        self._check(self._lib.omx_download(self._ctx, out.ctypes.data_as(C.c_void_p), C.c_void_p(t.ptr),
-                                           C.c_uint64(0), C.c_uint64(t.nbytes)))
+        _native.omx_download(self._context, out.ctypes.data, t, 0, t.nbytes)
         return out
 
     def download_f32(self, t: DeviceTensor) -> np.ndarray:
@@ -209,11 +177,11 @@ class MiBackend:
 
     def set_option(self, name: str, value: int):
         """Tuning knobs of the library (`omx_set_option`); no counterpart in the reference."""
-        self._check(self._lib.omx_set_option(self._ctx, name.encode(), C.c_int64(value)))
+        _native.omx_set_option(self._context, name.encode(), value)
 
     def sync(self):
         """BackendCore::sync (backend.rs:963-973)."""
-        self._check(self._lib.omx_sync(self._ctx))
+        _native.omx_sync(self._context)
 
     def _p(self, t: Optional[DeviceTensor]):
         return C.c_void_p(t.ptr) if t is not None else C.c_void_p(None)
@@ -221,17 +189,17 @@ class MiBackend:
     # ---- casts ----
     def cast_bf16(self, x: DeviceTensor) -> DeviceTensor:
         y = self.empty(x.shape, F32)
-        self._check(self._lib.omx_cast_bf16(self._ctx, self._p(x), self._p(y), C.c_uint64(x.numel)))
+        _native.omx_cast_bf16(self._context, x, y, x.numel)
         return y
 
     def to_bf16(self, x: DeviceTensor) -> DeviceTensor:
         y = self.empty(x.shape, BF16)
-        self._check(self._lib.omx_to_bf16(self._ctx, self._p(x), self._p(y), C.c_uint64(x.numel)))
+        _native.omx_to_bf16(self._context, x, y, x.numel)
         return y
 
     def to_f32(self, x: DeviceTensor) -> DeviceTensor:
         y = self.empty(x.shape, F32)
-        self._check(self._lib.omx_to_f32(self._ctx, self._p(x), self._p(y), C.c_uint64(x.numel)))
+        _native.omx_to_f32(self._context, x, y, x.numel)
         return y
 
     # ---- matmul class ----
@@ -242,9 +210,7 @@ class MiBackend:
             raise OjasError(SHAPE, f"linear_forward: input {x.shape} weight {w.shape}")
         od = F32 if out_dtype is None else out_dtype
         y = self.empty(x.shape[:-1] + (nout,), od)
-        self._check(self._lib.omx_linear_forward(self._ctx, self._p(x), C.c_int32(x.dtype), self._p(w),
-                                                 C.c_int32(w.dtype), self._p(y), C.c_int32(od), C.c_uint64(rows),
-                                                 C.c_uint64(kin), C.c_uint64(nout)))
+        _native.omx_linear_forward(self._context, x, x.dtype, w, w.dtype, y, od, rows, kin, nout)
         return y
 
     def linear_backward(self, x, w, gy, gx_dtype=F32, need_gx=True, need_gw=True):
@@ -254,73 +220,64 @@ class MiBackend:
             raise OjasError(DTYPE, "linear_backward: operands must share a dtype")
         gx = self.empty(x.shape, gx_dtype) if need_gx else None
         gw = self.empty(w.shape, F32) if need_gw else None
-        self._check(self._lib.omx_linear_backward(self._ctx, self._p(x), self._p(w), self._p(gy), C.c_int32(x.dtype),
-                                                  self._p(gx), C.c_int32(gx_dtype), self._p(gw), C.c_int32(F32),
-                                                  C.c_uint64(rows), C.c_uint64(kin), C.c_uint64(nout)))
+        _native.omx_linear_backward(self._context, x, w, gy, x.dtype, gx, gx_dtype, gw, F32, rows, kin, nout)
         return gx, gw
 
     def linear_backward_input(self, w, gy, in_features=None, gx_dtype=F32):
         rows = gy.numel // gy.shape[-1]
         kin, nout = w.shape[1], w.shape[0]
         gx = self.empty(gy.shape[:-1] + (kin,), gx_dtype)
-        self._check(self._lib.omx_linear_backward(self._ctx, None, self._p(w), self._p(gy), C.c_int32(w.dtype),
-                                                  self._p(gx), C.c_int32(gx_dtype), None, C.c_int32(F32),
-                                                  C.c_uint64(rows), C.c_uint64(kin), C.c_uint64(nout)))
+        _native.omx_linear_backward(self._context, None, w, gy, w.dtype, gx, gx_dtype, None, F32, rows, kin, nout)
         return gx
 
     def rope_half_split_inplace(self, x, cos, sin, tokens, time, heads, dim, backward=False):
         """The rotary embedding applied in place to the first heads * dim columns of bf16 x [tokens, pitch]."""
-        self._check(self._lib.omx_rope_half_split_inplace(
-            self._ctx, self._p(x), C.c_int32(x.dtype), C.c_uint64(x.shape[-1]), self._p(cos), self._p(sin),
-            C.c_uint64(tokens), C.c_uint64(time), C.c_uint64(heads), C.c_uint64(dim), C.c_int32(1 if backward else 0)))
+        _native.omx_rope_half_split_inplace(self._context, x, x.dtype, x.shape[-1], cos, sin, tokens, time, heads,
+                                            dim, (1 if backward else 0))
         return x
 
     def rope_half_split_pitched(self, x, cos, sin, tokens, time, heads, plain_heads, dim):
         """The rotation out of place: x [tokens, pitch] f32 or bf16 -> bf16, `heads` rotated heads then
         `plain_heads` converted as they are (`omx_rope_half_split_pitched`)."""
         out = self.empty(x.shape, BF16)
-        self._check(self._lib.omx_rope_half_split_pitched(
-            self._ctx, self._p(x), C.c_int32(x.dtype), self._p(out), C.c_uint64(x.shape[-1]), self._p(cos), self._p(sin),
-            C.c_uint64(tokens), C.c_uint64(time), C.c_uint64(heads), C.c_uint64(plain_heads), C.c_uint64(dim)))
+        _native.omx_rope_half_split_pitched(self._context, x, x.dtype, out, x.shape[-1], cos, sin, tokens, time,
+                                            heads, plain_heads, dim)
         return out
 
     def swiglu_forward(self, gate_up):
         rows, two_h = gate_up.shape
         out = self.empty((rows, two_h // 2), BF16)
-        self._check(self._lib.omx_swiglu_forward(self._ctx, self._p(gate_up), self._p(out), C.c_int32(gate_up.dtype),
-                                                 C.c_uint64(rows), C.c_uint64(two_h // 2)))
+        _native.omx_swiglu_forward(self._context, gate_up, out, gate_up.dtype, rows, two_h // 2)
         return out
 
     def swiglu_backward(self, gate_up, gy):
         rows, two_h = gate_up.shape
         g = self.empty(gate_up.shape, BF16)
-        self._check(self._lib.omx_swiglu_backward(self._ctx, self._p(gate_up), self._p(gy), self._p(g),
-                                                  C.c_int32(gate_up.dtype), C.c_uint64(rows), C.c_uint64(two_h // 2)))
+        _native.omx_swiglu_backward(self._context, gate_up, gy, g, gate_up.dtype, rows, two_h // 2)
         return g
 
     def pack_i8_group(self, codes, scales, group=32):
         """Row-major codes and scales -> the blocked layout (`omx_pack_i8_group`); same shapes."""
         nout, kin = codes.shape
         bc, bs = self.empty(codes.shape, I8), self.empty(scales.shape, F32)
-        self._check(self._lib.omx_pack_i8_group(self._ctx, self._p(codes), self._p(scales), self._p(bc), self._p(bs),
-                                                C.c_uint64(nout), C.c_uint64(kin), C.c_uint64(group), C.c_int32(0)))
+        _native.omx_pack_i8_group(self._context, codes, scales, bc, bs, nout, kin, group, 0)
         return bc, bs
 
     def unpack_i8_group(self, blocked_codes, blocked_scales, group=32):
         nout, kin = blocked_codes.shape
         c, s = self.empty(blocked_codes.shape, I8), self.empty(blocked_scales.shape, F32)
-        self._check(self._lib.omx_pack_i8_group(self._ctx, self._p(c), self._p(s), self._p(blocked_codes),
-                                                self._p(blocked_scales), C.c_uint64(nout), C.c_uint64(kin),
-                                                C.c_uint64(group), C.c_int32(1)))
+        _native.omx_pack_i8_group(self._context, c, s, blocked_codes, blocked_scales, nout, kin, group, 1)
         return c, s
 
     @staticmethod
     def _low_rank(low_rank):
-        """(h [rows, pitch] bf16, w [cols, rank] bf16, block_cols) -> a pointer to omx_low_rank, or None."""
+        """(h [rows, pitch] bf16, w [cols, rank] bf16, block_cols) -> an omx_low_rank and its address, or None
+        twice."""
         if low_rank is None:
-            return None
+            return None, None
         h, w, block_cols = low_rank
-        return C.byref(LowRank(h.ptr, w.ptr, h.shape[-1], w.shape[-1], w.shape[-1], block_cols))
+        tail = LowRank(h.ptr, w.ptr, h.shape[-1], w.shape[-1], w.shape[-1], block_cols)
+        return tail, C.addressof(tail)
 
     def linear_i8_group_forward(self, x, codes, scales, add=None, group=32, blocked=False, low_rank=None,
                                 out_dtype=BF16):
@@ -330,10 +287,9 @@ class MiBackend:
         if codes.shape != (nout, kin) or scales.shape != (nout, kin // group) or codes.dtype != I8 or scales.dtype != F32:
             raise OjasError(SHAPE, f"linear_i8_group_forward: input {x.shape} codes {codes.shape} scales {scales.shape}")
         y = self.empty(x.shape[:-1] + (nout,), out_dtype)
-        self._check(self._lib.omx_linear_i8_group_forward(
-            self._ctx, self._p(x), C.c_int32(x.dtype), self._p(codes), self._p(scales), C.c_uint64(group),
-            C.c_int32(1 if blocked else 0), self._p(add), self._low_rank(low_rank), self._p(y), C.c_int32(out_dtype),
-            C.c_uint64(rows), C.c_uint64(kin), C.c_uint64(nout)))
+        _tail, tail_at = self._low_rank(low_rank)  # the structure outlives the call
+        _native.omx_linear_i8_group_forward(self._context, x, x.dtype, codes, scales, group, (1 if blocked else 0),
+                                            add, tail_at, y, out_dtype, rows, kin, nout)
         return y
 
     def linear_i8_group_backward_input(self, codes, scales, gy, add=None, group=32, blocked=False, low_rank=None):
@@ -343,19 +299,17 @@ class MiBackend:
         if gy.shape[-1] != nout or scales.shape != (nout, kin // group) or codes.dtype != I8 or scales.dtype != F32:
             raise OjasError(SHAPE, f"linear_i8_group_backward_input: gy {gy.shape} codes {codes.shape}")
         gx = self.empty(gy.shape[:-1] + (kin,), BF16)
-        self._check(self._lib.omx_linear_i8_group_backward_input(
-            self._ctx, self._p(codes), self._p(scales), C.c_uint64(group), C.c_int32(1 if blocked else 0), self._p(gy),
-            C.c_int32(gy.dtype), self._p(add), self._low_rank(low_rank), self._p(gx), C.c_uint64(rows), C.c_uint64(kin), C.c_uint64(nout)))
+        _tail, tail_at = self._low_rank(low_rank)  # the structure outlives the call
+        _native.omx_linear_i8_group_backward_input(self._context, codes, scales, group, (1 if blocked else 0), gy,
+                                                   gy.dtype, add, tail_at, gx, rows, kin, nout)
         return gx
 
     def gemm(self, a: DeviceTensor, a_strides, b: DeviceTensor, b_strides, m, k, n, out_dtype=F32, c=None):
         """C[m,n] (+)= A.B with element strides (a_rs, a_cs), (b_rs, b_cs)."""
         acc = c is not None
         out = c if acc else self.empty((m, n), out_dtype)
-        self._check(self._lib.omx_gemm(self._ctx, self._p(a), C.c_uint64(a_strides[0]), C.c_uint64(a_strides[1]),
-                                       self._p(b), C.c_uint64(b_strides[0]), C.c_uint64(b_strides[1]),
-                                       C.c_int32(a.dtype), self._p(out), C.c_int32(out.dtype), C.c_uint64(m),
-                                       C.c_uint64(k), C.c_uint64(n), C.c_int32(1 if acc else 0)))
+        _native.omx_gemm(self._context, a, a_strides[0], a_strides[1], b, b_strides[0], b_strides[1], a.dtype, out,
+                         out.dtype, m, k, n, (1 if acc else 0))
         return out
 
     def gemm_strided_batch(self, a: DeviceTensor, a_strides, b: DeviceTensor, b_strides, m, k, n, count,
@@ -366,11 +320,8 @@ class MiBackend:
         if sc < m * n:
             raise OjasError(SHAPE, "gemm_strided_batch: outputs overlap")
         out = self.empty(((count - 1) * sc + m * n,), out_dtype)
-        self._check(self._lib.omx_gemm_strided_batch(
-            self._ctx, self._p(a), C.c_uint64(a_strides[0]), C.c_uint64(a_strides[1]), self._p(b),
-            C.c_uint64(b_strides[0]), C.c_uint64(b_strides[1]), C.c_int32(a.dtype), self._p(out), C.c_int32(out_dtype),
-            C.c_uint64(m), C.c_uint64(k), C.c_uint64(n), C.c_int32(0), C.c_uint64(count), C.c_uint64(sa),
-            C.c_uint64(sb), C.c_uint64(sc)))
+        _native.omx_gemm_strided_batch(self._context, a, a_strides[0], a_strides[1], b, b_strides[0], b_strides[1],
+                                       a.dtype, out, out_dtype, m, k, n, 0, count, sa, sb, sc)
         return out
 
     def gemm_pitched_strided_batch(self, a: DeviceTensor, a_strides, b: DeviceTensor, b_strides, c: DeviceTensor, ldc,
@@ -378,11 +329,8 @@ class MiBackend:
         """`gemm_strided_batch` into column blocks of `c`, whose rows are `ldc` elements apart
         (`omx_gemm_pitched_strided_batch`); writes `c` in place."""
         sa, sb, sc = batch_strides
-        self._check(self._lib.omx_gemm_pitched_strided_batch(
-            self._ctx, self._p(a), C.c_uint64(a_strides[0]), C.c_uint64(a_strides[1]), self._p(b),
-            C.c_uint64(b_strides[0]), C.c_uint64(b_strides[1]), C.c_int32(a.dtype), self._p(c), C.c_int32(c.dtype),
-            C.c_uint64(ldc), C.c_uint64(m), C.c_uint64(k), C.c_uint64(n), C.c_int32(0), C.c_uint64(count),
-            C.c_uint64(sa), C.c_uint64(sb), C.c_uint64(sc)))
+        _native.omx_gemm_pitched_strided_batch(self._context, a, a_strides[0], a_strides[1], b, b_strides[0],
+                                               b_strides[1], a.dtype, c, c.dtype, ldc, m, k, n, 0, count, sa, sb, sc)
 
     # ---- attention ----
     def causal_sdpa_forward(self, q, k, v, window: Optional[int] = None, out_dtype: Optional[int] = None):
@@ -393,10 +341,7 @@ class MiBackend:
         od = F32 if out_dtype is None else out_dtype
         out = self.empty(q.shape, od)
         lse = self.empty((b, h, t), F32)
-        self._check(self._lib.omx_causal_sdpa_forward(self._ctx, self._p(q), self._p(k), self._p(v),
-                                                      C.c_int32(q.dtype), self._p(out), C.c_int32(od), self._p(lse),
-                                                      C.c_uint64(b), C.c_uint64(h), C.c_uint64(hkv), C.c_uint64(t),
-                                                      C.c_uint64(d), C.c_uint64(window or 0)))
+        _native.omx_causal_sdpa_forward(self._context, q, k, v, q.dtype, out, od, lse, b, h, hkv, t, d, (window or 0))
         return out, lse
 
     def causal_sdpa_backward(self, q, k, v, out, lse, gy, window: Optional[int] = None, grad_dtype=F32):
@@ -410,12 +355,8 @@ class MiBackend:
         if out.shape != q.shape or gy.shape != q.shape or lse.dtype != F32:
             raise OjasError(SHAPE, f"causal_sdpa_backward: out {out.shape} / grad_output {gy.shape} against q {q.shape}")
         gq, gk, gv = self.empty(q.shape, grad_dtype), self.empty(k.shape, grad_dtype), self.empty(v.shape, grad_dtype)
-        self._check(self._lib.omx_causal_sdpa_backward(self._ctx, self._p(q), self._p(k), self._p(v), self._p(out),
-                                                       self._p(lse), self._p(gy), C.c_int32(q.dtype),
-                                                       C.c_int32(out.dtype), C.c_int32(gy.dtype), self._p(gq),
-                                                       self._p(gk), self._p(gv), C.c_int32(grad_dtype), C.c_uint64(b),
-                                                       C.c_uint64(h), C.c_uint64(hkv), C.c_uint64(t), C.c_uint64(d),
-                                                       C.c_uint64(window or 0)))
+        _native.omx_causal_sdpa_backward(self._context, q, k, v, out, lse, gy, q.dtype, out.dtype, gy.dtype, gq, gk,
+                                         gv, grad_dtype, b, h, hkv, t, d, (window or 0))
         return gq, gk, gv
 
     def causal_sdpa_backward_recompute(self, q, k, v, gy, window: Optional[int] = None, grad_dtype=F32):
@@ -427,19 +368,16 @@ class MiBackend:
         if gy.shape != q.shape:
             raise OjasError(SHAPE, f"causal_sdpa_backward_recompute: grad_output {gy.shape} against q {q.shape}")
         gq, gk, gv = self.empty(q.shape, grad_dtype), self.empty(k.shape, grad_dtype), self.empty(v.shape, grad_dtype)
-        self._check(self._lib.omx_causal_sdpa_backward_recompute(
-            self._ctx, self._p(q), self._p(k), self._p(v), self._p(gy), C.c_int32(q.dtype), C.c_int32(gy.dtype),
-            self._p(gq), self._p(gk), self._p(gv), C.c_int32(grad_dtype), C.c_uint64(b), C.c_uint64(h),
-            C.c_uint64(hkv), C.c_uint64(t), C.c_uint64(d), C.c_uint64(window or 0)))
+        _native.omx_causal_sdpa_backward_recompute(self._context, q, k, v, gy, q.dtype, gy.dtype, gq, gk, gv,
+                                                   grad_dtype, b, h, hkv, t, d, (window or 0))
         return gq, gk, gv
 
     def linear_gelu_forward(self, x, w, tanh_form: bool = False):
         """`linear_forward` then `gelu_*_forward` in one kernel (bf16): returns (u, gelu(u))."""
         rows, nout = x.numel // x.shape[-1], w.shape[0]
         u, act = self.empty(x.shape[:-1] + (nout,), BF16), self.empty(x.shape[:-1] + (nout,), BF16)
-        self._check(self._lib.omx_linear_gelu_forward(
-            self._ctx, self._p(x), self._p(w), C.c_int32(x.dtype), self._p(u), self._p(act), C.c_uint64(rows),
-            C.c_uint64(x.shape[-1]), C.c_uint64(nout), C.c_int32(1 if tanh_form else 0)))
+        _native.omx_linear_gelu_forward(self._context, x, w, x.dtype, u, act, rows, x.shape[-1], nout,
+                                        (1 if tanh_form else 0))
         return u, act
 
     def linear_backward_input_gelu(self, w, gy, u, tanh_form: bool = False):
@@ -447,11 +385,10 @@ class MiBackend:
         nout, nin = w.shape
         rows = gy.numel // nout
         if gy.shape[-1] != nout or u.numel != rows * nin or not (w.dtype == gy.dtype == u.dtype == BF16):
-            raise BackendError(OMX_SHAPE, f"linear_backward_input_gelu: w {w.shape}, gy {gy.shape}, u {u.shape}")
+            raise OjasError(SHAPE, f"linear_backward_input_gelu: w {w.shape}, gy {gy.shape}, u {u.shape}")
         gu = self.empty(u.shape, BF16)
-        self._check(self._lib.omx_linear_backward_input_gelu(
-            self._ctx, self._p(w), self._p(gy), C.c_int32(gy.dtype), self._p(u), self._p(gu), C.c_uint64(rows),
-            C.c_uint64(nin), C.c_uint64(nout), C.c_int32(1 if tanh_form else 0)))
+        _native.omx_linear_backward_input_gelu(self._context, w, gy, gy.dtype, u, gu, rows, nin, nout,
+                                               (1 if tanh_form else 0))
         return gu
 
     def causal_attention_forward(self, q, k, v, window: Optional[int] = None, pitches=None, saving: bool = False):
@@ -465,15 +402,13 @@ class MiBackend:
         qp, kvp = pitches if pitches else (h * d, hkv * d)
         out = self.empty((b, t, h, d), BF16)
         lse = self.empty((b, h, t), F32)
-        tail = (C.c_uint64(h * d), C.c_int32(BF16), self._p(lse), C.c_uint64(b), C.c_uint64(t), C.c_uint64(h),
-                C.c_uint64(hkv), C.c_uint64(d), C.c_uint64(window or 0))
-        head = (self._ctx, self._p(q), C.c_uint64(qp), self._p(k), self._p(v), C.c_uint64(kvp), C.c_int32(q.dtype),
-                self._p(out))
+        tail = (h * d, BF16, lse, b, t, h, hkv, d, window or 0)
+        head = (self._context, q, qp, k, v, kvp, q.dtype, out)
         if saving:
             residual = self.empty((b, t, h, d), BF16)
-            self._check(self._lib.omx_causal_attention_forward_saving(*head, self._p(residual), *tail))
+            _native.omx_causal_attention_forward_saving(*head, residual, *tail)
             return out, lse, residual
-        self._check(self._lib.omx_causal_attention_forward(*head, *tail))
+        _native.omx_causal_attention_forward(*head, *tail)
         return out, lse
 
     def causal_attention_backward(self, q, k, v, out, lse, gy, window: Optional[int] = None, pitches=None,
@@ -489,16 +424,14 @@ class MiBackend:
                 raise OjasError(SHAPE, "causal_attention_backward: pass `grads` with pitched operands")
             grads = (self.empty(q.shape, BF16), self.empty(k.shape, BF16), self.empty(v.shape, BF16))
         gq, gk, gv = grads
-        head = (self._ctx, self._p(q), C.c_uint64(qp), self._p(k), self._p(v), C.c_uint64(kvp), self._p(out))
-        tail = (self._p(gy), C.c_uint64(h * d), self._p(lse), C.c_int32(q.dtype), self._p(gq), self._p(gk), self._p(gv),
-                C.c_int32(BF16), C.c_uint64(b), C.c_uint64(t), C.c_uint64(h), C.c_uint64(hkv), C.c_uint64(d),
-                C.c_uint64(window or 0))
+        head = (self._context, q, qp, k, v, kvp, out)
+        tail = (gy, h * d, lse, q.dtype, gq, gk, gv, BF16, b, t, h, hkv, d, window or 0)
         if residual is not None:
             if residual.shape != out.shape or residual.dtype != BF16:
                 raise OjasError(SHAPE, "causal_attention_backward: residual must match the output")
-            self._check(self._lib.omx_causal_attention_backward_saved(*head, self._p(residual), *tail))
+            _native.omx_causal_attention_backward_saved(*head, residual, *tail)
         else:
-            self._check(self._lib.omx_causal_attention_backward(*head, *tail))
+            _native.omx_causal_attention_backward(*head, *tail)
         return gq, gk, gv
 
     # ---- norms ----
@@ -509,8 +442,7 @@ class MiBackend:
             raise OjasError(SHAPE, f"rms_norm_forward: weight {w.shape} for dim {dim}")
         od = x.dtype if out_dtype is None else out_dtype
         y = self.empty(x.shape, od)
-        self._check(self._lib.omx_rms_norm_forward(self._ctx, self._p(x), C.c_int32(x.dtype), self._p(w), self._p(y),
-                                                   C.c_int32(od), C.c_uint64(rows), C.c_uint64(dim), C.c_float(eps)))
+        _native.omx_rms_norm_forward(self._context, x, x.dtype, w, y, od, rows, dim, eps)
         return y
 
     def rms_norm_backward(self, x, w, gy, eps: float = 1e-6):
@@ -518,10 +450,7 @@ class MiBackend:
         rows = x.numel // dim
         gx = self.empty(x.shape, gy.dtype)
         gw = self.empty((dim,), F32)
-        self._check(self._lib.omx_rms_norm_backward(self._ctx, self._p(x), C.c_int32(x.dtype), self._p(w),
-                                                    self._p(gy), C.c_int32(gy.dtype), self._p(gx),
-                                                    C.c_int32(gy.dtype), self._p(gw), C.c_uint64(rows),
-                                                    C.c_uint64(dim), C.c_float(eps)))
+        _native.omx_rms_norm_backward(self._context, x, x.dtype, w, gy, gy.dtype, gx, gy.dtype, gw, rows, dim, eps)
         return gx, gw
 
     def residual_add_rms_norm_forward(self, x, y, w, eps: float = 1e-6, out_dtype: Optional[int] = None):
@@ -529,9 +458,8 @@ class MiBackend:
         dim = x.shape[-1]
         od = y.dtype if out_dtype is None else out_dtype
         total, normed = self.empty(x.shape, F32), self.empty(x.shape, od)
-        self._check(self._lib.omx_residual_add_rms_norm_forward(
-            self._ctx, self._p(x), C.c_int32(x.dtype), self._p(y), C.c_int32(y.dtype), self._p(w), self._p(total),
-            self._p(normed), C.c_int32(od), C.c_uint64(x.numel // dim), C.c_uint64(dim), C.c_float(eps)))
+        _native.omx_residual_add_rms_norm_forward(self._context, x, x.dtype, y, y.dtype, w, total, normed, od,
+                                                  x.numel // dim, dim, eps)
         return total, normed
 
     def rms_norm_backward_residual(self, x, w, gy, residual_grad, eps: float = 1e-6, want_bf16: bool = False,
@@ -542,24 +470,21 @@ class MiBackend:
         dim = x.shape[-1]
         gx, gw = self.empty(x.shape, F32), (self.empty((dim,), F32) if want_weight_grad else None)
         gx16 = self.empty(x.shape, BF16) if want_bf16 else None
-        self._check(self._lib.omx_rms_norm_backward_residual(
-            self._ctx, self._p(x), C.c_int32(x.dtype), self._p(w), self._p(gy), C.c_int32(gy.dtype),
-            self._p(residual_grad), self._p(gx), self._p(gx16), self._p(gw), C.c_uint64(x.numel // dim),
-            C.c_uint64(dim), C.c_float(eps)))
+        _native.omx_rms_norm_backward_residual(self._context, x, x.dtype, w, gy, gy.dtype, residual_grad, gx, gx16,
+                                               gw, x.numel // dim, dim, eps)
         return gx, gx16, gw
 
     # ---- loss ----
     @staticmethod
     def _ign(ignore_index):
-        return (C.c_int32(0), C.c_uint32(0)) if ignore_index is None else (C.c_int32(1), C.c_uint32(ignore_index))
+        return (0, 0) if ignore_index is None else (1, ignore_index)
 
     def cross_entropy_mean_forward(self, logits, targets, ignore_index=None):
         rows, vocab = logits.shape
         loss = self.empty((1,), F32)
         hi, iv = self._ign(ignore_index)
-        self._check(self._lib.omx_cross_entropy_mean_forward(self._ctx, self._p(logits), C.c_int32(logits.dtype),
-                                                             self._p(targets), C.c_uint64(rows), C.c_uint64(vocab),
-                                                             hi, iv, self._p(loss)))
+        _native.omx_cross_entropy_mean_forward(self._context, logits, logits.dtype, targets, rows, vocab, hi, iv,
+                                               loss)
         return loss
 
     def cross_entropy_mean_forward_static(self, logits, targets, loss, ignore_index=None):
@@ -567,18 +492,16 @@ class MiBackend:
         allocates nothing (row state in a file-scope device array; at most 65536 rows)."""
         rows, vocab = logits.shape
         hi, iv = self._ign(ignore_index)
-        self._check(self._lib.omx_cross_entropy_mean_forward_static(
-            self._ctx, self._p(logits), C.c_int32(logits.dtype), self._p(targets), C.c_uint64(rows),
-            C.c_uint64(vocab), hi, iv, self._p(loss)))
+        _native.omx_cross_entropy_mean_forward_static(self._context, logits, logits.dtype, targets, rows, vocab, hi,
+                                                      iv, loss)
         return loss
 
     def cross_entropy_mean_backward(self, logits, targets, ignore_index=None, grad_dtype=F32):
         rows, vocab = logits.shape
         grad = self.empty(logits.shape, grad_dtype)
         hi, iv = self._ign(ignore_index)
-        self._check(self._lib.omx_cross_entropy_mean_backward(self._ctx, self._p(logits), C.c_int32(logits.dtype),
-                                                              self._p(targets), C.c_uint64(rows), C.c_uint64(vocab),
-                                                              hi, iv, self._p(grad), C.c_int32(grad_dtype)))
+        _native.omx_cross_entropy_mean_backward(self._context, logits, logits.dtype, targets, rows, vocab, hi, iv,
+                                                grad, grad_dtype)
         return grad
 
     def linear_cross_entropy_mean(self, x, w, targets, ignore_index=None, chunk=(1024, 8192), grads=(True, True),
@@ -592,10 +515,8 @@ class MiBackend:
         gx = self.empty(x.shape, gx_dtype) if grads[0] else None
         gw = self.empty(w.shape, F32) if grads[1] else None
         hi, iv = self._ign(ignore_index)
-        self._check(self._lib.omx_linear_cross_entropy_mean(
-            self._ctx, self._p(x), self._p(w), C.c_int32(x.dtype), self._p(targets), C.c_uint64(rows),
-            C.c_uint64(dim), C.c_uint64(vocab), hi, iv, C.c_uint64(chunk[0]), C.c_uint64(chunk[1]), self._p(loss),
-            self._p(gx), C.c_int32(gx_dtype), self._p(gw)))
+        _native.omx_linear_cross_entropy_mean(self._context, x, w, x.dtype, targets, rows, dim, vocab, hi, iv,
+                                              chunk[0], chunk[1], loss, gx, gx_dtype, gw)
         return loss, gx, gw
 
     # ---- embedding ----
@@ -603,17 +524,13 @@ class MiBackend:
         vocab, dim = table.shape
         od = F32 if out_dtype is None else out_dtype
         out = self.empty(ids.shape + (dim,), od)
-        self._check(self._lib.omx_embedding_forward(self._ctx, self._p(table), C.c_int32(table.dtype), self._p(ids),
-                                                    self._p(out), C.c_int32(od), C.c_uint64(ids.numel),
-                                                    C.c_uint64(vocab), C.c_uint64(dim)))
+        _native.omx_embedding_forward(self._context, table, table.dtype, ids, out, od, ids.numel, vocab, dim)
         return out
 
     def embedding_backward(self, ids, grad, vocab: int):
         dim = grad.shape[-1]
         out = self.empty((vocab, dim), F32)
-        self._check(self._lib.omx_embedding_backward(self._ctx, self._p(ids), self._p(grad), C.c_int32(grad.dtype),
-                                                     self._p(out), C.c_uint64(ids.numel), C.c_uint64(vocab),
-                                                     C.c_uint64(dim)))
+        _native.omx_embedding_backward(self._context, ids, grad, grad.dtype, out, ids.numel, vocab, dim)
         return out
 
     def embedding_backward_accumulate(self, ids, grad, table_grad):
@@ -622,31 +539,26 @@ class MiBackend:
         vocab, dim = table_grad.shape
         if table_grad.dtype != F32 or grad.shape[-1] != dim:
             raise OjasError(SHAPE, f"embedding_backward_accumulate: grad {grad.shape} against table_grad {table_grad.shape}")
-        self._check(self._lib.omx_embedding_backward_accumulate(
-            self._ctx, self._p(ids), self._p(grad), C.c_int32(grad.dtype), self._p(table_grad), C.c_uint64(ids.numel),
-            C.c_uint64(vocab), C.c_uint64(dim)))
+        _native.omx_embedding_backward_accumulate(self._context, ids, grad, grad.dtype, table_grad, ids.numel, vocab,
+                                                  dim)
 
     # ---- optimizers (in place) ----
     def adamw_step(self, param, grad, moment1, moment2, step: int, config: AdamWConfig, param_bf16=None):
-        self._check(self._lib.omx_adamw_step(self._ctx, self._p(param), self._p(grad), self._p(moment1),
-                                             self._p(moment2), C.c_uint64(param.numel), C.c_uint64(step),
-                                             C.byref(config), self._p(param_bf16)))
+        _native.omx_adamw_step(self._context, param, grad, moment1, moment2, param.numel, step, C.addressof(config),
+                               param_bf16)
 
     def adamw_step_bounded(self, param, grad, moment1, moment2, step: int, config: AdamWConfig, inputs_bounded: bool,
                            unbounded_flag: DeviceTensor, param_bf16=None):
         """`adamw_step` for a caller that tracks its tensors between calls: with `inputs_bounded`
         (every input below 2^60 in magnitude) the checking pass is skipped; `unbounded_flag` (one
         u32) is OR-ed with 1 when a stored parameter or moment reaches 2^60."""
-        self._check(self._lib.omx_adamw_step_bounded(
-            self._ctx, self._p(param), self._p(grad), self._p(moment1), self._p(moment2), C.c_uint64(param.numel),
-            C.c_uint64(step), C.byref(config), self._p(param_bf16), C.c_int32(1 if inputs_bounded else 0),
-            self._p(unbounded_flag)))
+        _native.omx_adamw_step_bounded(self._context, param, grad, moment1, moment2, param.numel, step,
+                                       C.addressof(config), param_bf16, (1 if inputs_bounded else 0), unbounded_flag)
 
     def muon_ns5_step(self, param, grad, momentum, config: MuonNs5Config, param_bf16=None):
         rows, cols = param.shape
-        self._check(self._lib.omx_muon_ns5_step(self._ctx, self._p(param), self._p(grad), self._p(momentum),
-                                                C.c_uint64(rows), C.c_uint64(cols), C.byref(config),
-                                                self._p(param_bf16)))
+        _native.omx_muon_ns5_step(self._context, param, grad, momentum, rows, cols, C.addressof(config),
+                                  param_bf16)
 
     def muon_ns5_step_batched(self, params, grads, momenta, config: MuonNs5Config, params_bf16=None):
         """`muon_ns5_step` on several tensors of one shape in one set of launches (in place)."""
@@ -656,17 +568,16 @@ class MiBackend:
             raise OjasError(SHAPE, "muon_ns5_step_batched: tensors of one shape, one gradient and momentum each")
         table = lambda ts: (C.c_void_p * n)(*[t.ptr for t in ts])
         mirrors = (C.c_void_p * n)(*[(t.ptr if t is not None else None) for t in params_bf16]) if params_bf16 else None
-        self._check(self._lib.omx_muon_ns5_step_batched(self._ctx, table(params), table(grads), table(momenta), mirrors,
-                                                        C.c_uint64(n), C.c_uint64(rows), C.c_uint64(cols),
-                                                        C.byref(config)))
+        tables = [table(ts) for ts in (params, grads, momenta)] + ([mirrors] if mirrors is not None else [])
+        _native.omx_muon_ns5_step_batched(self._context, *([C.addressof(t) for t in tables] + [None])[:4], n, rows, cols,
+                                          C.addressof(config))
 
     def clip_grad_norm(self, grads: Sequence[DeviceTensor], max_norm: float) -> float:
         n = len(grads)
         ptrs = (C.c_void_p * max(n, 1))(*[g.ptr for g in grads])
         lens = (C.c_uint64 * max(n, 1))(*[g.numel for g in grads])
         norm = C.c_float()
-        self._check(self._lib.omx_clip_grad_norm(self._ctx, ptrs, lens, C.c_uint64(n), C.c_float(max_norm),
-                                                 C.byref(norm)))
+        _native.omx_clip_grad_norm(self._context, C.addressof(ptrs), C.addressof(lens), n, max_norm, C.addressof(norm))
         return float(norm.value)
 
     # ---- elementwise / layout ----
@@ -675,26 +586,23 @@ class MiBackend:
             raise OjasError(SHAPE, "residual_add_forward: operands differ")
         od = x.dtype if out_dtype is None else out_dtype
         out = self.empty(x.shape, od)
-        self._check(self._lib.omx_residual_add(self._ctx, self._p(x), C.c_int32(x.dtype), self._p(y),
-                                               C.c_int32(y.dtype), self._p(out), C.c_int32(od), C.c_uint64(x.numel)))
+        _native.omx_residual_add(self._context, x, x.dtype, y, y.dtype, out, od, x.numel)
         return out
 
     def accumulate_grad(self, acc, grad):
-        self._check(self._lib.omx_accumulate_grad(self._ctx, self._p(acc), self._p(grad), C.c_uint64(acc.numel)))
+        _native.omx_accumulate_grad(self._context, acc, grad, acc.numel)
 
     def scale_grad(self, grad, scale: float):
-        self._check(self._lib.omx_scale_grad(self._ctx, self._p(grad), C.c_float(scale), C.c_uint64(grad.numel)))
+        _native.omx_scale_grad(self._context, grad, scale, grad.numel)
 
     def _gelu(self, x, tanh_form):
         y = self.empty(x.shape, x.dtype)
-        self._check(self._lib.omx_gelu_forward(self._ctx, self._p(x), self._p(y), C.c_int32(x.dtype),
-                                               C.c_uint64(x.numel), C.c_int32(tanh_form)))
+        _native.omx_gelu_forward(self._context, x, y, x.dtype, x.numel, tanh_form)
         return y
 
     def _gelu_bwd(self, x, gy, tanh_form):
         gx = self.empty(x.shape, x.dtype)
-        self._check(self._lib.omx_gelu_backward(self._ctx, self._p(x), self._p(gy), self._p(gx), C.c_int32(x.dtype),
-                                                C.c_uint64(x.numel), C.c_int32(tanh_form)))
+        _native.omx_gelu_backward(self._context, x, gy, gx, x.dtype, x.numel, tanh_form)
         return gx
 
     def gelu_erf_forward(self, x):
@@ -714,8 +622,7 @@ class MiBackend:
             raise OjasError(UNSUPPORTED, "permute: only axes [0,2,1,3] of a rank-4 tensor")
         d0, d1, d2, d3 = x.shape
         y = self.empty((d0, d2, d1, d3), x.dtype)
-        self._check(self._lib.omx_permute_0213(self._ctx, self._p(x), self._p(y), C.c_int32(x.dtype), C.c_uint64(d0),
-                                               C.c_uint64(d1), C.c_uint64(d2), C.c_uint64(d3)))
+        _native.omx_permute_0213(self._context, x, y, x.dtype, d0, d1, d2, d3)
         return y
 
     # ---- ops of the nanolab block (backend.rs:1151-1163,1674-1708,1860-1920) ----
@@ -729,29 +636,25 @@ class MiBackend:
 
     def silu_forward(self, x):
         y = self.empty(x.shape, x.dtype)
-        self._check(self._lib.omx_silu_forward(self._ctx, self._p(x), self._p(y), C.c_int32(x.dtype),
-                                               C.c_uint64(x.numel)))
+        _native.omx_silu_forward(self._context, x, y, x.dtype, x.numel)
         return y
 
     def silu_backward(self, x, gy):
         self._same("silu_backward", x, gy)
         gx = self.empty(x.shape, x.dtype)
-        self._check(self._lib.omx_silu_backward(self._ctx, self._p(x), self._p(gy), self._p(gx), C.c_int32(x.dtype),
-                                                C.c_uint64(x.numel)))
+        _native.omx_silu_backward(self._context, x, gy, gx, x.dtype, x.numel)
         return gx
 
     def mul_forward(self, a, b):
         self._same("mul_forward", a, b)
         out = self.empty(a.shape, a.dtype)
-        self._check(self._lib.omx_mul_forward(self._ctx, self._p(a), self._p(b), self._p(out), C.c_int32(a.dtype),
-                                              C.c_uint64(a.numel)))
+        _native.omx_mul_forward(self._context, a, b, out, a.dtype, a.numel)
         return out
 
     def mul_backward(self, a, b, gy):
         self._same("mul_backward", a, b, gy)
         ga, gb = self.empty(a.shape, a.dtype), self.empty(a.shape, a.dtype)
-        self._check(self._lib.omx_mul_backward(self._ctx, self._p(a), self._p(b), self._p(gy), self._p(ga),
-                                               self._p(gb), C.c_int32(a.dtype), C.c_uint64(a.numel)))
+        _native.omx_mul_backward(self._context, a, b, gy, ga, gb, a.dtype, a.numel)
         return ga, gb
 
     def _rope(self, fn, op, x, cos, sin):
@@ -770,15 +673,14 @@ class MiBackend:
         else:
             raise OjasError(SHAPE, f"{op}: cos/sin shape {cos.shape} does not broadcast onto {x.shape}")
         y = self.empty(x.shape, x.dtype)
-        self._check(fn(self._ctx, self._p(x), self._p(cos), self._p(sin), self._p(y), C.c_int32(x.dtype),
-                       C.c_uint64(rows), C.c_uint64(dim), C.c_uint64(time), C.c_uint64(heads)))
+        fn(self._context, x, cos, sin, y, x.dtype, rows, dim, time, heads)
         return y
 
     def rope_half_split_forward(self, x, cos, sin):
-        return self._rope(self._lib.omx_rope_half_split_forward, "rope_half_split_forward", x, cos, sin)
+        return self._rope(_native.omx_rope_half_split_forward, "rope_half_split_forward", x, cos, sin)
 
     def rope_half_split_backward(self, grad_output, cos, sin):
-        return self._rope(self._lib.omx_rope_half_split_backward, "rope_half_split_backward", grad_output, cos, sin)
+        return self._rope(_native.omx_rope_half_split_backward, "rope_half_split_backward", grad_output, cos, sin)
 
     def rms_qk_norm_forward(self, q, k, q_weight, k_weight, eps: float = 1e-6, out_dtype: Optional[int] = None):
         dim = q.shape[-1]
@@ -787,10 +689,8 @@ class MiBackend:
                                    f"{k_weight.shape}")
         od = q.dtype if out_dtype is None else out_dtype
         qn, kn = self.empty(q.shape, od), self.empty(k.shape, od)
-        self._check(self._lib.omx_rms_qk_norm_forward(
-            self._ctx, self._p(q), self._p(k), C.c_int32(q.dtype), self._p(q_weight), self._p(k_weight), self._p(qn),
-            self._p(kn), C.c_int32(od), C.c_uint64(q.numel // dim), C.c_uint64(k.numel // dim), C.c_uint64(dim),
-            C.c_float(eps)))
+        _native.omx_rms_qk_norm_forward(self._context, q, k, q.dtype, q_weight, k_weight, qn, kn, od, q.numel // dim,
+                                        k.numel // dim, dim, eps)
         return qn, kn
 
     def rms_qk_norm_backward(self, q, k, q_weight, k_weight, grad_q, grad_k, eps: float = 1e-6):
@@ -799,11 +699,9 @@ class MiBackend:
             raise OjasError(SHAPE, "rms_qk_norm_backward: gradient shapes do not match q / k")
         gq, gk = self.empty(q.shape, grad_q.dtype), self.empty(k.shape, grad_q.dtype)
         gqw, gkw = self.empty((dim,), F32), self.empty((dim,), F32)
-        self._check(self._lib.omx_rms_qk_norm_backward(
-            self._ctx, self._p(q), self._p(k), C.c_int32(q.dtype), self._p(q_weight), self._p(k_weight),
-            self._p(grad_q), self._p(grad_k), C.c_int32(grad_q.dtype), self._p(gq), self._p(gk),
-            C.c_int32(grad_q.dtype), self._p(gqw), self._p(gkw), C.c_uint64(q.numel // dim),
-            C.c_uint64(k.numel // dim), C.c_uint64(dim), C.c_float(eps)))
+        _native.omx_rms_qk_norm_backward(self._context, q, k, q.dtype, q_weight, k_weight, grad_q, grad_k,
+                                         grad_q.dtype, gq, gk, grad_q.dtype, gqw, gkw, q.numel // dim, k.numel // dim,
+                                         dim, eps)
         return gq, gk, gqw, gkw
 
     def _gate_dims(self, op, x, w, b, attn):
@@ -826,10 +724,8 @@ class MiBackend:
         od = attn.dtype if out_dtype is None else out_dtype
         y = self.empty(attn.shape, od)
         gates = self.empty((rows, heads), F32) if save else None
-        self._check(self._lib.omx_per_head_sigmoid_gate_forward(
-            self._ctx, self._p(x), self._p(w), C.c_int32(x.dtype), self._p(b), self._p(attn), C.c_int32(attn.dtype),
-            self._p(y), C.c_int32(od), self._p(gates), C.c_uint64(rows), C.c_uint64(d_model), C.c_uint64(heads),
-            C.c_uint64(dh)))
+        _native.omx_per_head_sigmoid_gate_forward(self._context, x, w, x.dtype, b, attn, attn.dtype, y, od, gates,
+                                                  rows, d_model, heads, dh)
         return y, gates
 
     def per_head_sigmoid_gate_forward(self, x, w, b, attn, out_dtype: Optional[int] = None):
@@ -845,11 +741,8 @@ class MiBackend:
         gxd = x.dtype if g_input_dtype is None else g_input_dtype
         gx, gw = self.empty(x.shape, gxd), self.empty(w.shape, F32)
         gb, ga = self.empty((heads,), F32), self.empty(attn.shape, attn.dtype)
-        self._check(self._lib.omx_per_head_sigmoid_gate_backward(
-            self._ctx, self._p(x), self._p(w), C.c_int32(x.dtype), self._p(b), self._p(attn), C.c_int32(attn.dtype),
-            self._p(gy), C.c_int32(gy.dtype), self._p(scales), self._p(gx), C.c_int32(gxd), self._p(gw), self._p(gb),
-            self._p(ga), C.c_int32(attn.dtype), C.c_uint64(rows), C.c_uint64(d_model), C.c_uint64(heads),
-            C.c_uint64(dh)))
+        _native.omx_per_head_sigmoid_gate_backward(self._context, x, w, x.dtype, b, attn, attn.dtype, gy, gy.dtype,
+                                                   scales, gx, gxd, gw, gb, ga, attn.dtype, rows, d_model, heads, dh)
         return gx, gw, gb, ga
 
     def per_head_sigmoid_gate_backward(self, x, w, b, attn, gy, g_input_dtype: Optional[int] = None):
@@ -864,9 +757,8 @@ class MiBackend:
             raise OjasError(SHAPE, f"per_head_sigmoid_gate_input_grad_add: gz {gz.shape}, weight {w.shape}, "
                                    f"add_in {add_in.shape}")
         out = self.empty(add_in.shape, F32)
-        self._check(self._lib.omx_per_head_sigmoid_gate_input_grad_add(
-            self._ctx, self._p(gz), self._p(w), C.c_int32(w.dtype), self._p(add_in), C.c_int32(add_in.dtype),
-            self._p(out), C.c_uint64(rows), C.c_uint64(d_model), C.c_uint64(heads)))
+        _native.omx_per_head_sigmoid_gate_input_grad_add(self._context, gz, w, w.dtype, add_in, add_in.dtype, out,
+                                                         rows, d_model, heads)
         return out
 
     def per_head_sigmoid_gate_backward_deferred(self, x, w, b, attn, gy, scales, g_input_dtype: Optional[int] = None,
@@ -885,11 +777,9 @@ class MiBackend:
         gx = self.empty(x.shape, gxd) if want_input_grad else None
         gz = self.empty((rows, heads), x.dtype)
         gb, ga = self.empty((heads,), F32), self.empty(attn.shape, attn.dtype)
-        self._check(self._lib.omx_per_head_sigmoid_gate_backward_deferred(
-            self._ctx, self._p(x), self._p(w), C.c_int32(x.dtype), self._p(b), self._p(attn), C.c_int32(attn.dtype),
-            self._p(gy), C.c_int32(gy.dtype), self._p(scales), self._p(gx), C.c_int32(gxd), self._p(gz), self._p(gb),
-            self._p(ga), C.c_int32(attn.dtype), C.c_uint64(rows), C.c_uint64(d_model), C.c_uint64(heads),
-            C.c_uint64(dh)))
+        _native.omx_per_head_sigmoid_gate_backward_deferred(self._context, x, w, x.dtype, b, attn, attn.dtype, gy,
+                                                            gy.dtype, scales, gx, gxd, gz, gb, ga, attn.dtype, rows,
+                                                            d_model, heads, dh)
         return gx, gz, gb, ga
 
     def qkv_prepare_forward(self, qkv_lin, q_weight, k_weight, cos, sin, heads, kv_heads, head_dim, value0=None, lam=None,
@@ -900,10 +790,8 @@ class MiBackend:
         if value0 is not None and value0.dtype != qkv_lin.dtype:
             raise OjasError(DTYPE, "qkv_prepare_forward: value0 has the projection output's dtype")
         out = self.empty(qkv_lin.shape, BF16)
-        self._check(self._lib.omx_qkv_prepare_forward(
-            self._ctx, self._p(qkv_lin), C.c_int32(qkv_lin.dtype), self._p(out), C.c_uint64(pitch), self._p(q_weight), self._p(k_weight),
-            self._p(cos), self._p(sin), self._p(value0), self._p(lam), C.c_uint64(b * t), C.c_uint64(t), C.c_uint64(heads),
-            C.c_uint64(kv_heads), C.c_uint64(head_dim), C.c_float(eps)))
+        _native.omx_qkv_prepare_forward(self._context, qkv_lin, qkv_lin.dtype, out, pitch, q_weight, k_weight, cos,
+                                        sin, value0, lam, b * t, t, heads, kv_heads, head_dim, eps)
         return out
 
     def qkv_prepare_backward(self, qkv_lin, g_qkv, q_weight, k_weight, cos, sin, heads, kv_heads, head_dim, value0=None,
@@ -916,11 +804,10 @@ class MiBackend:
         g_lin = self.empty(qkv_lin.shape, BF16)
         gqw, gkw = self.empty((head_dim,), F32), self.empty((head_dim,), F32)
         g_lam = self.empty((1,), F32) if value0 is not None else None
-        self._check(self._lib.omx_qkv_prepare_backward(
-            self._ctx, self._p(qkv_lin), C.c_int32(qkv_lin.dtype), self._p(g_qkv), self._p(g_lin), C.c_uint64(pitch), self._p(q_weight),
-            self._p(k_weight), self._p(cos), self._p(sin), self._p(value0), self._p(lam), self._p(value0_grad),
-            C.c_int32(1 if value0_grad_first else 0), self._p(add_value_grad), self._p(gqw), self._p(gkw), self._p(g_lam),
-            C.c_uint64(b * t), C.c_uint64(t), C.c_uint64(heads), C.c_uint64(kv_heads), C.c_uint64(head_dim), C.c_float(eps)))
+        _native.omx_qkv_prepare_backward(self._context, qkv_lin, qkv_lin.dtype, g_qkv, g_lin, pitch, q_weight,
+                                         k_weight, cos, sin, value0, lam, value0_grad,
+                                         (1 if value0_grad_first else 0), add_value_grad, gqw, gkw, g_lam, b * t, t,
+                                         heads, kv_heads, head_dim, eps)
         return g_lin, gqw, gkw, g_lam
 
     def value_residual_blend_forward(self, value, value0, lam):
@@ -928,9 +815,7 @@ class MiBackend:
         if lam.numel != 1 or lam.dtype != F32:
             raise OjasError(SHAPE, "value_residual_blend_forward: lambda must be one f32")
         out = self.empty(value.shape, value.dtype)
-        self._check(self._lib.omx_value_residual_blend_forward(
-            self._ctx, self._p(value), self._p(value0), self._p(lam), self._p(out), C.c_int32(value.dtype),
-            C.c_uint64(value.numel)))
+        _native.omx_value_residual_blend_forward( self._context, value, value0, lam, out, value.dtype, value.numel)
         return out
 
     def value_residual_blend_backward(self, value, value0, lam, gy):
@@ -939,9 +824,8 @@ class MiBackend:
             raise OjasError(SHAPE, "value_residual_blend_backward: lambda must be one f32")
         gv, gv0 = self.empty(value.shape, value.dtype), self.empty(value.shape, value.dtype)
         gl = self.empty((1,), F32)
-        self._check(self._lib.omx_value_residual_blend_backward(
-            self._ctx, self._p(value), self._p(value0), self._p(lam), self._p(gy), self._p(gv), self._p(gv0),
-            C.c_int32(value.dtype), self._p(gl), C.c_uint64(value.numel)))
+        _native.omx_value_residual_blend_backward(self._context, value, value0, lam, gy, gv, gv0, value.dtype, gl,
+                                                  value.numel)
         return gv, gv0, gl
 
     # ---- integer ops ----
@@ -959,10 +843,8 @@ class MiBackend:
         if q.dtype != F32 or k_cache.dtype != v_cache.dtype:
             raise OjasError(DTYPE, "cached_attention_forward: q is f32 and the caches share a dtype")
         out = self.empty(q.shape, F32)
-        self._check(self._lib.omx_cached_attention_forward(
-            self._ctx, self._p(q), self._p(k_cache), self._p(v_cache), C.c_int32(k_cache.dtype), self._p(out),
-            C.c_uint64(b), C.c_uint64(tq), C.c_uint64(h), C.c_uint64(hkv), C.c_uint64(d), C.c_uint64(cap),
-            C.c_uint64(kv_len), C.c_uint64(window or 0)))
+        _native.omx_cached_attention_forward(self._context, q, k_cache, v_cache, k_cache.dtype, out, b, tq, h, hkv, d,
+                                             cap, kv_len, (window or 0))
         return out
 
     def kv_cache_write(self, cache, src, at: int):
@@ -975,9 +857,7 @@ class MiBackend:
             raise OjasError(SHAPE, f"kv_cache_write: src {src.shape} does not fit cache {cache.shape}")
         if src.dtype != F32:
             raise OjasError(DTYPE, "kv_cache_write: src is f32")
-        self._check(self._lib.omx_kv_cache_write(self._ctx, self._p(cache), C.c_int32(cache.dtype), self._p(src),
-                                                 C.c_uint64(b), C.c_uint64(cap), C.c_uint64(hkv), C.c_uint64(d),
-                                                 C.c_uint64(tn), C.c_uint64(at)))
+        _native.omx_kv_cache_write(self._context, cache, cache.dtype, src, b, cap, hkv, d, tn, at)
 
     def token_windows(self, tokens: DeviceTensor, starts, seq_len: int):
         """(x, y) u32 [batch, seq_len] from a bin resident on the device (`upload` of
@@ -986,22 +866,20 @@ class MiBackend:
         starts = np.ascontiguousarray(starts, np.uint64)
         batch = int(starts.size)
         x, y = self.empty((batch, seq_len), U32), self.empty((batch, seq_len), U32)
-        self._check(self._lib.omx_token_windows(self._ctx, self._p(tokens), C.c_int32(_SIZE_OF[tokens.dtype]),
-                                                C.c_uint64(tokens.numel), starts.ctypes.data_as(C.c_void_p),
-                                                C.c_uint64(batch), C.c_uint64(seq_len), self._p(x), self._p(y)))
+        _native.omx_token_windows(self._context, tokens, _SIZE_OF[tokens.dtype], tokens.numel, starts.ctypes.data, batch,
+                                  seq_len, x, y)
         return x, y
 
     def argmax_rows(self, x):
         rows, cols = x.shape
         out = self.empty((rows,), U32)
-        self._check(self._lib.omx_argmax_rows(self._ctx, self._p(x), C.c_uint64(rows), C.c_uint64(cols), self._p(out)))
+        _native.omx_argmax_rows(self._context, x, rows, cols, out)
         return out
 
     def topk_rows(self, x, k: int):
         rows, cols = x.shape
         vals, ids = self.empty((rows, k), F32), self.empty((rows, k), U32)
-        self._check(self._lib.omx_topk_rows(self._ctx, self._p(x), C.c_uint64(rows), C.c_uint64(cols), C.c_uint64(k),
-                                            self._p(vals), self._p(ids)))
+        _native.omx_topk_rows(self._context, x, rows, cols, k, vals, ids)
         return vals, ids
 
     def __getattr__(self, name):
@@ -1091,7 +969,7 @@ def _shape_first(name, method, validator, operands):
         except shapes.ShapeError as e:
             raise OjasError(e.code, f"{e.op}: {e.detail}") from None
         for t in args[:operands]:
-            if t is not None and not isinstance(t, DeviceTensor):
+            if type(t) is not DeviceTensor and t is not None:
                 raise OjasError(PLACEMENT, f"{name}: operand is in host memory")
         return method(self, *args, **kwargs)
 

@@ -1,0 +1,467 @@
+// Python's side of the C ABI in native code: the device tensor `MiBackend` hands out and a typed call
+// for every entry point its methods make.
+//
+// What bounds a decode step or an op-by-op training step of a small model is this path, not the
+// device: some 170 calls per decoded token. Through ctypes a call boxed each argument in an object of
+// its own, allocated and freed its output through two more calls and took 12-15 us of host time for
+// a 2-5 us kernel. Here an argument is converted straight into the parameter's type (deduced from the
+// declaration in ojas_mi355x.h, so there is no second table of signatures), and a tensor's
+// allocation, release and views are C.
+//
+// The library is opened at run time (`load`), so importing this module needs neither it nor a device.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <dlfcn.h>
+#include <structmember.h>
+
+#include <cstring>
+#include <tuple>
+#include <type_traits>
+#include <utility>
+
+#include "ojas_mi355x.h"
+
+namespace {
+
+PyObject* g_error = nullptr;  // OjasError(code, detail)
+constexpr int kSizes[4] = {4, 2, 4, 1};  // F32, BF16, U32, I8
+
+// ---- the context: an omx_ctx whose handle becomes null when the backend closes ----
+struct Context {
+  PyObject_HEAD
+  omx_ctx* ctx;
+};
+
+int32_t (*p_alloc)(omx_ctx*, uint64_t, void**) = nullptr;
+int32_t (*p_free)(omx_ctx*, void*) = nullptr;
+size_t (*p_last_error)(omx_ctx*, char*, size_t) = nullptr;
+
+PyObject* raise(omx_ctx* ctx, int32_t rc) {
+  char buf[512];
+  buf[0] = 0;
+  if (ctx && p_last_error) p_last_error(ctx, buf, sizeof buf);
+  PyObject* text = PyUnicode_DecodeUTF8(buf, static_cast<Py_ssize_t>(strlen(buf)), "replace");
+  if (!text) return nullptr;
+  PyObject* e = PyObject_CallFunction(g_error ? g_error : PyExc_RuntimeError, "iN", static_cast<int>(rc), text);
+  if (!e) return nullptr;
+  PyErr_SetObject(reinterpret_cast<PyObject*>(Py_TYPE(e)), e);
+  Py_DECREF(e);
+  return nullptr;
+}
+
+PyObject* raise_text(int32_t rc, const char* text) {
+  PyObject* e = PyObject_CallFunction(g_error ? g_error : PyExc_RuntimeError, "is", static_cast<int>(rc), text);
+  if (!e) return nullptr;
+  PyErr_SetObject(reinterpret_cast<PyObject*>(Py_TYPE(e)), e);
+  Py_DECREF(e);
+  return nullptr;
+}
+
+PyObject* context_new(PyTypeObject* type, PyObject* args, PyObject*) {
+  unsigned long long address = 0;
+  if (!PyArg_ParseTuple(args, "K", &address)) return nullptr;
+  Context* self = reinterpret_cast<Context*>(type->tp_alloc(type, 0));
+  if (self) self->ctx = reinterpret_cast<omx_ctx*>(address);
+  return reinterpret_cast<PyObject*>(self);
+}
+PyObject* context_close(PyObject* self, PyObject*) {
+  reinterpret_cast<Context*>(self)->ctx = nullptr;
+  Py_RETURN_NONE;
+}
+PyMethodDef context_methods[] = {{"close", context_close, METH_NOARGS, "Forget the handle; tensors no longer free themselves."},
+                                 {nullptr, nullptr, 0, nullptr}};
+PyTypeObject ContextType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ---- the device tensor ----
+struct Tensor {
+  PyObject_HEAD
+  Context* context;   // whose device memory this is
+  PyObject* backend;  // the MiBackend (None once dropped)
+  PyObject* shape;    // tuple of int
+  PyObject* base;     // the tensor a view keeps alive
+  unsigned long long ptr;
+  Py_ssize_t numel;
+  int dtype;
+  char owns, compute_bf16;
+};
+PyTypeObject TensorType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// Elements of a shape tuple (1 for rank 0); -1 with an error set when an axis is no whole number.
+Py_ssize_t elements(PyObject* shape) {
+  Py_ssize_t n = 1;
+  const Py_ssize_t rank = PyTuple_GET_SIZE(shape);
+  for (Py_ssize_t i = 0; i < rank; ++i) {
+    const Py_ssize_t axis = PyLong_AsSsize_t(PyTuple_GET_ITEM(shape, i));
+    if (axis == -1 && PyErr_Occurred()) return -1;
+    n *= axis;
+  }
+  return n;
+}
+
+// A tuple of plain ints from a shape given as a tuple, a list or one number.
+PyObject* shape_tuple(PyObject* given) {
+  if (PyTuple_CheckExact(given)) {
+    const Py_ssize_t rank = PyTuple_GET_SIZE(given);
+    bool plain = true;
+    for (Py_ssize_t i = 0; i < rank; ++i) plain &= PyLong_CheckExact(PyTuple_GET_ITEM(given, i)) != 0;
+    if (plain) {
+      Py_INCREF(given);
+      return given;
+    }
+  }
+  PyObject* seq = PyIndex_Check(given) ? PyTuple_Pack(1, given) : PySequence_Tuple(given);
+  if (!seq) return nullptr;
+  PyObject* out = PyTuple_New(PyTuple_GET_SIZE(seq));
+  for (Py_ssize_t i = 0; out && i < PyTuple_GET_SIZE(seq); ++i) {
+    PyObject* axis = PyNumber_Long(PyTuple_GET_ITEM(seq, i));
+    if (!axis) Py_CLEAR(out);
+    else PyTuple_SET_ITEM(out, i, axis);
+  }
+  Py_DECREF(seq);
+  return out;
+}
+
+Tensor* make_tensor(PyObject* backend, Context* context, unsigned long long ptr, PyObject* shape /* stolen */, Py_ssize_t n,
+                    int dtype, bool owns) {
+  Tensor* t = reinterpret_cast<Tensor*>(TensorType.tp_alloc(&TensorType, 0));
+  if (!t) {
+    Py_DECREF(shape);
+    return nullptr;
+  }
+  Py_XINCREF(context);
+  Py_INCREF(backend);
+  t->context = context;
+  t->backend = backend;
+  t->shape = shape;
+  t->ptr = ptr;
+  t->numel = n;
+  t->dtype = dtype;
+  t->owns = owns;
+  return t;
+}
+
+// DeviceTensor(backend, ptr, shape, dtype, owns=True)
+PyObject* tensor_new(PyTypeObject*, PyObject* args, PyObject* kwargs) {
+  static const char* names[] = {"backend", "ptr", "shape", "dtype", "owns", nullptr};
+  PyObject *backend, *ptr_obj, *given;
+  int dtype, owns = 1;
+  if (!PyArg_ParseTupleAndKeywords(args, kwargs, "OOOi|p", const_cast<char**>(names), &backend, &ptr_obj, &given, &dtype, &owns))
+    return nullptr;
+  unsigned long long ptr = 0;
+  if (ptr_obj != Py_None) {
+    ptr = PyLong_AsUnsignedLongLong(ptr_obj);
+    if (PyErr_Occurred()) return nullptr;
+  }
+  PyObject* context = backend == Py_None ? nullptr : PyObject_GetAttrString(backend, "_context");
+  if (!context) PyErr_Clear();
+  if (context && Py_TYPE(context) != &ContextType) Py_CLEAR(context);
+  PyObject* shape = shape_tuple(given);
+  if (!shape) {
+    Py_XDECREF(context);
+    return nullptr;
+  }
+  const Py_ssize_t n = elements(shape);
+  Tensor* t = n == -1 && PyErr_Occurred() ? nullptr
+                                          : make_tensor(backend, reinterpret_cast<Context*>(context), ptr, shape, n, dtype, owns);
+  Py_XDECREF(context);
+  return reinterpret_cast<PyObject*>(t);
+}
+
+void tensor_dealloc(PyObject* self) {
+  Tensor* t = reinterpret_cast<Tensor*>(self);
+  PyObject_GC_UnTrack(self);
+  if (t->owns && t->ptr && t->context && t->context->ctx && p_free) {
+    // A block too large for the context's pool goes back to the driver, which waits for the stream.
+    PyThreadState* unlocked = t->numel >= (64l << 20) ? PyEval_SaveThread() : nullptr;
+    p_free(t->context->ctx, reinterpret_cast<void*>(t->ptr));
+    if (unlocked) PyEval_RestoreThread(unlocked);
+  }
+  Py_XDECREF(t->context);
+  Py_XDECREF(t->backend);
+  Py_XDECREF(t->shape);
+  Py_XDECREF(t->base);
+  Py_TYPE(self)->tp_free(self);
+}
+int tensor_traverse(PyObject* self, visitproc visit, void* arg) {
+  Tensor* t = reinterpret_cast<Tensor*>(self);
+  Py_VISIT(t->backend);
+  Py_VISIT(t->base);
+  return 0;
+}
+int tensor_clear(PyObject* self) {
+  Tensor* t = reinterpret_cast<Tensor*>(self);
+  Py_CLEAR(t->base);
+  PyObject* backend = t->backend;
+  Py_INCREF(Py_None);
+  t->backend = Py_None;
+  Py_XDECREF(backend);
+  return 0;
+}
+
+PyObject* tensor_nbytes(PyObject* self, void*) {
+  const Tensor* t = reinterpret_cast<const Tensor*>(self);
+  return PyLong_FromSsize_t(t->numel * ((t->dtype >= 0 && t->dtype < 4) ? kSizes[t->dtype] : 0));
+}
+
+// reshape(*shape) or reshape(shape): a zero-copy view (tensor.rs:1555-1605) that does not own the memory.
+PyObject* tensor_reshape(PyObject* self, PyObject* args) {
+  Tensor* t = reinterpret_cast<Tensor*>(self);
+  PyObject* given = args;
+  if (PyTuple_GET_SIZE(args) == 1 && (PyTuple_Check(PyTuple_GET_ITEM(args, 0)) || PyList_Check(PyTuple_GET_ITEM(args, 0))))
+    given = PyTuple_GET_ITEM(args, 0);
+  PyObject* shape = shape_tuple(given);
+  if (!shape) return nullptr;
+  const Py_ssize_t n = elements(shape);
+  if (n != t->numel) {
+    if (!PyErr_Occurred()) {
+      PyObject* text = PyUnicode_FromFormat("reshape %R -> %R", t->shape, shape);
+      if (text) raise_text(OMX_SHAPE, PyUnicode_AsUTF8(text));
+      Py_XDECREF(text);
+    }
+    Py_DECREF(shape);
+    return nullptr;
+  }
+  Tensor* view = make_tensor(t->backend, t->context, t->ptr, shape, n, t->dtype, false);
+  if (!view) return nullptr;
+  Py_INCREF(self);
+  view->base = self;
+  view->compute_bf16 = t->compute_bf16;
+  return reinterpret_cast<PyObject*>(view);
+}
+
+PyMethodDef tensor_methods[] = {{"reshape", tensor_reshape, METH_VARARGS, "A zero-copy view of another shape."},
+                                {nullptr, nullptr, 0, nullptr}};
+PyMemberDef tensor_members[] = {
+    {"backend", T_OBJECT, offsetof(Tensor, backend), READONLY, nullptr},
+    {"shape", T_OBJECT, offsetof(Tensor, shape), READONLY, nullptr},
+    {"ptr", T_ULONGLONG, offsetof(Tensor, ptr), 0, nullptr},
+    {"dtype", T_INT, offsetof(Tensor, dtype), READONLY, nullptr},
+    {"numel", T_PYSSIZET, offsetof(Tensor, numel), READONLY, nullptr},
+    {"_owns", T_BOOL, offsetof(Tensor, owns), 0, nullptr},
+    {"_base", T_OBJECT, offsetof(Tensor, base), READONLY, nullptr},
+    // The storage compute tag of an f32 tensor (tensor.rs COMPUTE_BF16): true when its values are known
+    // to be bf16-exact, so a second rounding would only clone. Set by `Autocast`.
+    {"compute_bf16", T_BOOL, offsetof(Tensor, compute_bf16), 0, nullptr},
+    {nullptr, 0, 0, 0, nullptr}};
+PyGetSetDef tensor_getset[] = {{"nbytes", tensor_nbytes, nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+
+// empty(backend, context, shape, dtype): a new tensor charged to the context's budget.
+PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 4 || Py_TYPE(args[1]) != &ContextType) {
+    PyErr_SetString(PyExc_TypeError, "empty(backend, context, shape, dtype)");
+    return nullptr;
+  }
+  Context* c = reinterpret_cast<Context*>(args[1]);
+  const long dtype = PyLong_AsLong(args[3]);
+  if (dtype == -1 && PyErr_Occurred()) return nullptr;
+  if (dtype < 0 || dtype > 3) {
+    PyErr_SetObject(PyExc_KeyError, args[3]);
+    return nullptr;
+  }
+  PyObject* shape = shape_tuple(args[2]);
+  if (!shape) return nullptr;
+  const Py_ssize_t n = elements(shape);
+  if (n == -1 && PyErr_Occurred()) {
+    Py_DECREF(shape);
+    return nullptr;
+  }
+  void* p = nullptr;
+  const int32_t rc = c->ctx && p_alloc ? p_alloc(c->ctx, static_cast<uint64_t>(n > 1 ? n : 1) * kSizes[dtype], &p) : OMX_BACKEND;
+  if (rc != OMX_OK) {
+    Py_DECREF(shape);
+    return raise(c->ctx, rc);
+  }
+  Tensor* t = make_tensor(args[0], c, reinterpret_cast<unsigned long long>(p), shape, n, static_cast<int>(dtype), true);
+  if (!t) p_free(c->ctx, p);
+  return reinterpret_cast<PyObject*>(t);
+}
+
+// ---- typed calls ----
+// One argument converted into parameter type T. A pointer is a tensor's memory, null or a plain
+// address; a host array is refused (its address would reach a kernel).
+template <typename T>
+bool convert(PyObject* o, T* out) {
+  if constexpr (std::is_same_v<T, omx_ctx*>) {
+    if (Py_TYPE(o) != &ContextType) {
+      PyErr_SetString(PyExc_TypeError, "the first argument is the backend's context");
+      return false;
+    }
+    *out = reinterpret_cast<Context*>(o)->ctx;
+    return true;
+  } else if constexpr (std::is_pointer_v<T>) {
+    if (Py_TYPE(o) == &TensorType) {
+      *out = reinterpret_cast<T>(reinterpret_cast<Tensor*>(o)->ptr);
+      return true;
+    }
+    if (o == Py_None) {
+      *out = nullptr;
+      return true;
+    }
+    if (PyLong_Check(o)) {
+      const unsigned long long v = PyLong_AsUnsignedLongLong(o);
+      *out = reinterpret_cast<T>(v);
+      return !(v == static_cast<unsigned long long>(-1) && PyErr_Occurred());
+    }
+    if (std::is_same_v<T, const char*> && PyBytes_Check(o)) {
+      *out = reinterpret_cast<T>(PyBytes_AS_STRING(o));
+      return true;
+    }
+    PyErr_Format(PyExc_TypeError, "a device tensor is expected, not %.80s", Py_TYPE(o)->tp_name);
+    return false;
+  } else if constexpr (std::is_floating_point_v<T>) {
+    const double v = PyFloat_AsDouble(o);
+    *out = static_cast<T>(v);
+    return !(v == -1.0 && PyErr_Occurred());
+  } else if constexpr (std::is_signed_v<T>) {
+    const long long v = PyLong_AsLongLong(o);
+    *out = static_cast<T>(v);
+    if (v == -1 && PyErr_Occurred()) return false;
+    if (static_cast<long long>(*out) != v) {
+      PyErr_SetString(PyExc_OverflowError, "argument out of range");
+      return false;
+    }
+    return true;
+  } else {
+    PyObject* whole = PyNumber_Index(o);
+    if (!whole) return false;
+    const unsigned long long v = PyLong_AsUnsignedLongLong(whole);
+    Py_DECREF(whole);
+    *out = static_cast<T>(v);
+    if (v == static_cast<unsigned long long>(-1) && PyErr_Occurred()) return false;
+    if (static_cast<unsigned long long>(*out) != v) {
+      PyErr_SetString(PyExc_OverflowError, "argument out of range");
+      return false;
+    }
+    return true;
+  }
+}
+
+// Entry<ID, Signature>: the function's address (filled by `load`) and the Python callable around it.
+template <int ID, typename F>
+struct Entry;
+template <int ID, typename... P>
+struct Entry<ID, int32_t(P...)> {
+  static inline int32_t (*address)(P...) = nullptr;
+
+  template <size_t... I>
+  static PyObject* invoke(PyObject* const* args, std::index_sequence<I...>) {
+    std::tuple<P...> v;
+    if (!(convert(args[I], &std::get<I>(v)) && ...)) return nullptr;
+    int32_t rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = address(std::get<I>(v)...);
+    Py_END_ALLOW_THREADS
+    if (rc != OMX_OK) return raise(std::get<0>(v), rc);
+    Py_RETURN_NONE;
+  }
+  static PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != static_cast<Py_ssize_t>(sizeof...(P)) || !address) {
+      PyErr_Format(PyExc_TypeError, address ? "%zu arguments expected" : "the library is not loaded", sizeof...(P));
+      return nullptr;
+    }
+    return invoke(args, std::make_index_sequence<sizeof...(P)>{});
+  }
+};
+
+struct Symbol {
+  const char* name;
+  void** address;
+};
+
+#define OMX_ENTRIES(X)                                                                                                   \
+  X(omx_fill_zero) X(omx_upload) X(omx_download) X(omx_sync) X(omx_cast_bf16) X(omx_to_bf16) X(omx_to_f32)               \
+  X(omx_linear_forward) X(omx_linear_backward) X(omx_gemm) X(omx_gemm_strided_batch) X(omx_gemm_pitched_strided_batch)   \
+  X(omx_linear_i8_group_forward) X(omx_linear_i8_group_backward_input) X(omx_pack_i8_group)                              \
+  X(omx_causal_sdpa_forward) X(omx_causal_sdpa_backward) X(omx_causal_sdpa_backward_recompute)                           \
+  X(omx_linear_gelu_forward) X(omx_linear_backward_input_gelu) X(omx_causal_attention_forward)                           \
+  X(omx_causal_attention_backward) X(omx_causal_attention_forward_saving) X(omx_causal_attention_backward_saved)         \
+  X(omx_rms_norm_forward) X(omx_rms_norm_backward) X(omx_residual_add_rms_norm_forward)                                  \
+  X(omx_rms_norm_backward_residual) X(omx_cross_entropy_mean_forward) X(omx_cross_entropy_mean_forward_static)           \
+  X(omx_cross_entropy_mean_backward) X(omx_linear_cross_entropy_mean) X(omx_embedding_forward) X(omx_embedding_backward) \
+  X(omx_embedding_backward_accumulate) X(omx_adamw_step) X(omx_adamw_step_bounded) X(omx_muon_ns5_step)                  \
+  X(omx_muon_ns5_step_batched) X(omx_clip_grad_norm) X(omx_residual_add) X(omx_accumulate_grad) X(omx_scale_grad)        \
+  X(omx_gelu_forward) X(omx_gelu_backward) X(omx_cached_attention_forward) X(omx_kv_cache_write) X(omx_token_windows)    \
+  X(omx_permute_0213) X(omx_silu_forward) X(omx_silu_backward) X(omx_mul_forward) X(omx_mul_backward)                    \
+  X(omx_rope_half_split_forward) X(omx_rope_half_split_backward) X(omx_rope_half_split_inplace)                          \
+  X(omx_rope_half_split_pitched) X(omx_swiglu_forward) X(omx_swiglu_backward) X(omx_rms_qk_norm_forward)                 \
+  X(omx_rms_qk_norm_backward) X(omx_per_head_sigmoid_gate_forward) X(omx_per_head_sigmoid_gate_backward)                 \
+  X(omx_per_head_sigmoid_gate_backward_deferred) X(omx_per_head_sigmoid_gate_input_grad_add)                             \
+  X(omx_value_residual_blend_forward) X(omx_value_residual_blend_backward) X(omx_qkv_prepare_forward)                    \
+  X(omx_qkv_prepare_backward) X(omx_argmax_rows) X(omx_topk_rows) X(omx_set_option)
+
+enum EntryId {
+#define X(name) ID_##name,
+  OMX_ENTRIES(X)
+#undef X
+};
+#define X(name) {#name, reinterpret_cast<void**>(&Entry<ID_##name, decltype(::name)>::address)},
+Symbol g_symbols[] = {OMX_ENTRIES(X)};
+#undef X
+
+// load(path, error_type): opens the library and finds every entry point.
+PyObject* load(PyObject*, PyObject* args) {
+  const char* path;
+  PyObject* error;
+  if (!PyArg_ParseTuple(args, "sO", &path, &error)) return nullptr;
+  Py_INCREF(error);
+  Py_XDECREF(g_error);
+  g_error = error;
+  if (p_alloc) Py_RETURN_NONE;
+  void* lib = dlopen(path, RTLD_NOW | RTLD_LOCAL);
+  if (!lib) return raise_text(OMX_BACKEND, dlerror());
+  auto find = [&](const char* name) {
+    void* p = dlsym(lib, name);
+    if (!p) raise_text(OMX_BACKEND, name);
+    return p;
+  };
+  for (const Symbol& s : g_symbols)
+    if (!(*s.address = find(s.name))) return nullptr;
+  void* alloc = find("omx_alloc");
+  if (!alloc || !(p_free = reinterpret_cast<decltype(p_free)>(find("omx_free"))) ||
+      !(p_last_error = reinterpret_cast<decltype(p_last_error)>(find("omx_last_error"))))
+    return nullptr;
+  p_alloc = reinterpret_cast<decltype(p_alloc)>(alloc);
+  Py_RETURN_NONE;
+}
+
+#define X(name) \
+  {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Entry<ID_##name, decltype(::name)>::call)), METH_FASTCALL, nullptr},
+PyMethodDef module_methods[] = {
+    OMX_ENTRIES(X){"load", load, METH_VARARGS, "load(path, error_type)"},
+    {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&empty)), METH_FASTCALL, "empty(backend, context, shape, dtype)"},
+    {nullptr, nullptr, 0, nullptr}};
+#undef X
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Typed calls into libojas_mi355x and its device tensor.", -1, module_methods,
+                      nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) {
+  ContextType.tp_name = "ojas_amd._native.Context";
+  ContextType.tp_basicsize = sizeof(Context);
+  ContextType.tp_flags = Py_TPFLAGS_DEFAULT;
+  ContextType.tp_new = context_new;
+  ContextType.tp_methods = context_methods;
+  TensorType.tp_name = "ojas_amd._native.DeviceTensor";
+  TensorType.tp_doc =
+      "A contiguous device tensor: pointer, shape, dtype. Frees itself on drop\n"
+      "(the role of `Arc<dyn DeviceBuffer>` + `Reservation`, tensor.rs:146-163).";
+  TensorType.tp_basicsize = sizeof(Tensor);
+  TensorType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  TensorType.tp_new = tensor_new;
+  TensorType.tp_dealloc = tensor_dealloc;
+  TensorType.tp_traverse = tensor_traverse;
+  TensorType.tp_clear = tensor_clear;
+  TensorType.tp_methods = tensor_methods;
+  TensorType.tp_members = tensor_members;
+  TensorType.tp_getset = tensor_getset;
+  if (PyType_Ready(&ContextType) < 0 || PyType_Ready(&TensorType) < 0) return nullptr;
+  PyObject* m = PyModule_Create(&module);
+  if (!m) return nullptr;
+  Py_INCREF(&ContextType);
+  Py_INCREF(&TensorType);
+  if (PyModule_AddObject(m, "Context", reinterpret_cast<PyObject*>(&ContextType)) < 0 ||
+      PyModule_AddObject(m, "DeviceTensor", reinterpret_cast<PyObject*>(&TensorType)) < 0)
+    return nullptr;
+  return m;
+}

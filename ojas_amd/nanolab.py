@@ -80,6 +80,12 @@ class NanolabGraph:
 
     def __init__(self, be: MiBackend, spec: NanolabSpec, params: Dict[str, DeviceTensor]):
         self.be, self.spec, self.p = be, spec, params
+        self._rope = (0, None, None)  # (sequence length, cos, sin): the tables of the last length, on the device
+
+    def _rope_tables(self, seq: int):
+        if self._rope[0] != seq:
+            self._rope = (seq, *(self.be.upload(t) for t in rope_tables(self.spec, seq)))
+        return self._rope[1:]
 
     def _blk(self, i: int, name: str) -> DeviceTensor:
         return self.p[f"blocks.{i}.{name}"]
@@ -92,8 +98,7 @@ class NanolabGraph:
         B, T = ids.shape
         N, d, H, KV, D = B * T, s.n_embd, s.n_head, s.n_kv_head, s.head_dim
         eps, win = s.rms_eps, s.window
-        cos_h, sin_h = rope_tables(s, T)
-        cos, sin = be.upload(cos_h), be.upload(sin_h)
+        cos, sin = self._rope_tables(T)
         swap = [0, 2, 1, 3]
 
         # ---- forward (block.rs:218-264) ----

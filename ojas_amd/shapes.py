@@ -37,13 +37,20 @@ class ShapeError(Exception):
 
 def dtype_of(t) -> int:
     d = t.dtype
-    if isinstance(d, int):
+    if type(d) is int:
         return d
     return _NUMPY.get(np.dtype(d), -1)
 
 
 def shape_of(t) -> Tuple[int, ...]:
-    return tuple(int(x) for x in t.shape)
+    return t.shape  # a tuple of ints, of a device tensor and of a numpy array alike
+
+
+def _product(axes) -> int:
+    n = 1
+    for a in axes:
+        n *= a
+    return n
 
 
 def _refuse(op, detail):
@@ -54,10 +61,10 @@ def _operand(op, t, allowed) -> int:
     """shapes.rs:411-431 `operand`: dtype, then no zero axis; returns the element count."""
     if dtype_of(t) not in allowed:
         raise ShapeError(DTYPE, op, f"dtype {dtype_of(t)} where {allowed} is expected")
-    s = shape_of(t)
-    if 0 in s:
+    n = _product(t.shape)
+    if n == 0:
         raise _refuse(op, "empty tensor")
-    return int(np.prod(s, dtype=np.int64)) if s else 1
+    return n
 
 
 def _float(op, t) -> int:
@@ -69,7 +76,7 @@ def _u32(op, t) -> int:
 
 
 def _same(op, a, b):
-    if tuple(a) != tuple(b):
+    if a != b:
         raise _refuse(op, f"shape {list(a)} does not match {list(b)}")
 
 
@@ -80,7 +87,7 @@ def _same_shape(op, tensors) -> int:
     first = shape_of(tensors[0])
     for t in tensors[1:]:
         _same(op, first, shape_of(t))
-    return int(np.prod(first, dtype=np.int64)) if first else 1
+    return _product(first)
 
 
 def _split_last(op, shape, rank0):
@@ -90,7 +97,7 @@ def _split_last(op, shape, rank0):
 
 
 def _rows(lead) -> int:
-    return int(np.prod(lead, dtype=np.int64)) if lead else 1
+    return _product(lead)
 
 
 # ---- integer ops: shapes.rs:503-547
@@ -238,15 +245,14 @@ def _sdpa(op, q, k, v):
         raise _refuse(op, f"sdpa query rank {len(qs)} != 4 [B, H, T, D]")
     if ks != vs:
         raise _refuse(op, f"sdpa k {list(ks)} and v {list(vs)} differ")
-    differ = _refuse(op, f"sdpa shapes q {list(qs)} k {list(ks)} v {list(vs)} differ")
     if len(ks) != 4:
-        raise differ
+        raise _refuse(op, f"sdpa shapes q {list(qs)} k {list(ks)} v {list(vs)} differ")
     batch, heads, seq, dim = qs
     kb, kv_heads, kseq, kd = ks
     grouped = kv_heads != heads
     if (kb, kseq, kd) != (batch, seq, dim) or (grouped and (kv_heads == 0 or heads == 0 or kv_heads > heads or
                                                             heads % kv_heads)):
-        raise differ
+        raise _refuse(op, f"sdpa shapes q {list(qs)} k {list(ks)} v {list(vs)} differ")
     return batch, heads, kv_heads, seq, dim
 
 
