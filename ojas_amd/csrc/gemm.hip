@@ -473,8 +473,11 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   // own kernel, which neither tiles the output nor splits K across launches.
   const bool thin = operand_dtype == OMX_BF16 && ctx->gemm_thin && !(epi && epi->mode != OMX_EPI_NONE) &&
                     omx_gemm_thin_eligible(g, a_km, b_km);
+  // Few rows (a decoder's linear layers): K shared between a workgroup's waves, no tile of 128 rows.
+  const bool skinny = operand_dtype == OMX_BF16 && !thin && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0 &&
+                      omx_gemm_skinny_eligible(ctx, g, a_km, b_km);
   int dma_variant = -1;
-  if (!thin && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km)) {
+  if (!thin && !skinny && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km)) {
     const int mode = ctx->gemm_dma_mode;
     if (mode == 1 && ctx->gemm_forced_tiling >= 0) {
       dma_variant = ctx->gemm_forced_tiling;
@@ -604,7 +607,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     // 108 tiles: two splits; of 2304 x 768, 324 tiles: two splits make three rounds of half the length).
     const long all_tiles = tiles * g.batches;
     const bool may_split =
-        !thin && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
+        !thin && !skinny && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
     if (may_split && ksteps >= 4 * min_steps && !(epi && epi->mode != OMX_EPI_NONE)) {
       splits = static_cast<int>(((g.batches == 1 ? 512 : 1024) + all_tiles - 1) / all_tiles);
       if (splits > ksteps / min_steps) splits = ksteps / min_steps;
@@ -676,6 +679,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   int32_t rc;
   if (thin) {
     rc = omx_gemm_thin_launch(ctx, g, b_km);
+  } else if (skinny) {
+    rc = omx_gemm_skinny_launch(ctx, g);
   } else if (dma_variant >= 0) {
     rc = omx_gemm_dma_launch(ctx, g, a_km, b_km, dma_variant);
     if (rc == OMX_OK && g.splits > 1) {

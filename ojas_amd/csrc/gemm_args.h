@@ -280,3 +280,7 @@ int32_t omx_gemm_dma_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_k
 // (K a multiple of 128, no accumulation): one pass over A, no split-K reduce.
 bool omx_gemm_thin_eligible(const GemmArgs& g, bool a_km, bool b_km);
 int32_t omx_gemm_thin_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km);
+
+// bf16 kernel for products of few rows or few outputs, both operands k-contiguous, K a multiple of 32.
+bool omx_gemm_skinny_eligible(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km);
+int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);

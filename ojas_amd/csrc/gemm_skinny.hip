@@ -1,0 +1,149 @@
+// bf16 product with few rows: C[M, N] = A.B with A [M, K] and B's columns [N, K] both k-contiguous (a decoder's
+// linear layers on one token per sequence, or on a short prompt chunk). Same contract as gemm.hip
+// (f32 accumulation; reference: ojas-cpu/src/linalg.rs:69-210).
+//
+// Such a product reads N x K of weights for 2 M operations per value: it is bound by reading the
+// weights once, and with a few hundred KiB of them by one round of memory latency and the launch. The
+// 128-row tiles of the other kernels leave all but N / 128 compute units idle and run their K loop as
+// a serial chain of loads, barriers and products. Here a workgroup owns 16 NB columns and up to 64
+// rows, and its waves share K between them: both operands go from memory straight into
+// v_mfma_f32_16x16x32_bf16 fragments (a lane's eight k-consecutive values are one 16-byte load; no
+// LDS, no barrier in the loop), CHUNK steps' loads are in flight together, and the waves'
+// partial sums meet in LDS in wave order: one launch, no split-K pass.
+#include "gemm_tiles.h"
+
+namespace {
+
+typedef __bf16 bf16x8_s __attribute__((ext_vector_type(8)));
+typedef float floatx4_s __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4_s __attribute__((ext_vector_type(4)));
+
+
+
+// MB x NB blocks of 16 rows x 16 columns per workgroup.
+template <int MB, int NB, int WAVES, int CHUNK>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(GemmArgs g) {
+  extern __shared__ float skinny_red[];  // [WAVES][MB * NB][4][64]
+  gemm_select_batch(g, blockIdx.z);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, kc = (lane >> 4) * 8;
+  const int row0 = blockIdx.y * (16 * MB), col0 = blockIdx.x * (16 * NB);
+  // Rows and columns past the end are read from the last one and never stored.
+  const unsigned short* a[MB];
+  const unsigned short* b[NB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+    a[m] = static_cast<const unsigned short*>(g.a) + static_cast<long>(min(row0 + m * 16 + l16, g.M - 1)) * g.lda + kc;
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+    b[n] = static_cast<const unsigned short*>(g.b) + static_cast<long>(min(col0 + n * 16 + l16, g.N - 1)) * g.ldb + kc;
+  floatx4_s acc[MB][NB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[m][n] = floatx4_s{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int steps = g.K / 32;
+  const int s_end = steps * (wave + 1) / WAVES;
+  for (int s0 = steps * wave / WAVES; s0 < s_end; s0 += CHUNK) {
+    const int live = min(CHUNK, s_end - s0);  // uniform over the wave
+    u32x4_s bf[CHUNK][NB], af[CHUNK][MB];
+#pragma unroll
+    for (int s = 0; s < CHUNK; ++s) {
+      if (s < live) {
+        const long k = static_cast<long>(s0 + s) * 32;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) bf[s][n] = *reinterpret_cast<const u32x4_s*>(b[n] + k);
+#pragma unroll
+        for (int m = 0; m < MB; ++m) af[s][m] = *reinterpret_cast<const u32x4_s*>(a[m] + k);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < CHUNK; ++s)
+      if (s < live)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int m = 0; m < MB; ++m)
+            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_s, bf[s][n]),
+                                                                __builtin_bit_cast(bf16x8_s, af[s][m]), acc[m][n], 0, 0, 0);
+  }
+  // acc[m][n][v] is row m * 16 + l16, column n * 16 + 4 * (lane / 16) + v of this wave's share of K.
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) skinny_red[((wave * (MB * NB) + m * NB + n) * 4 + v) * 64 + lane] = acc[m][n][v];
+  __syncthreads();
+  bool bad = false;
+  for (int blk = wave; blk < MB * NB; blk += WAVES) {
+    const int row = row0 + blk / NB * 16 + l16, col = col0 + blk % NB * 16 + (lane >> 4) * 4;
+    float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[v] += skinny_red[((w * (MB * NB) + blk) * 4 + v) * 64 + lane];
+    if (row < g.M && col < g.N)
+      bad |= g.epi == OMX_EPI_NONE ? gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3])
+                                   : gemm_store4_epi(g, 0, row, col, x[0], x[1], x[2], x[3]);
+  }
+  if (bad) dev_raise_fault(g.fault, g.tag);
+}
+
+struct SkinnyTile {
+  int mb, nb;
+};
+constexpr SkinnyTile SKINNY_TILES[] = {{1, 1}, {1, 2}, {2, 2}, {4, 4}};
+constexpr int SKINNY_WAVES = 8, SKINNY_CHUNK = 4;
+
+// The smallest tile that makes at most one workgroup per compute unit: a workgroup's time is its own
+// operand rows (2.5 us + about 1 ns per column of K and 16-row block: a CU fetches 64-byte row pieces at
+// some 65 GB/s), so a bigger tile pays only when it saves a second round of workgroups. Beyond
+// K (MB + NB) = 18000, some 20 us, splitting K over the chip and adding up in a second launch is as fast
+// (768 columns over K = 3072: 13 against 19 us at 256 rows, 25 against 20 at 512). At most 32 rows of any
+// width: the weights are nearly all there is to read, so the tile follows the rows and the columns run in as
+// many rounds as they need (50304 columns over K = 768, one row: 14.4 us = 5.4 TB/s). -1: neither.
+// One row, 768 x 768: 15.2 -> 3.2 us; 64 rows: 16.6 -> 3.8; 1024 rows: 19.3 -> 9.4 with their split pass.
+int skinny_tile(const GemmArgs& g, long units) {
+  const long m = (g.M + 15) / 16, n = (g.N + 15) / 16;
+  for (int t = 0; t < 4; ++t) {
+    const SkinnyTile tile = SKINNY_TILES[t];
+    const long groups = ((m + tile.mb - 1) / tile.mb) * ((n + tile.nb - 1) / tile.nb);
+    if (groups * g.batches <= units) return static_cast<long>(g.K) * (tile.mb + tile.nb) <= 18000 ? t : -1;
+  }
+  if (g.K > 4096) return -1;
+  if (g.M <= 4) return 0;
+  if (g.M <= 16) return 1;
+  if (g.M <= 32) return 2;
+  return -1;
+}
+
+template <int MB, int NB>
+int32_t launch_skinny(omx_ctx* ctx, const GemmArgs& g) {
+  constexpr int smem = SKINNY_WAVES * MB * NB * 1024;
+  auto kernel = &gemm_skinny_kernel<MB, NB, SKINNY_WAVES, SKINNY_CHUNK>;
+  if constexpr (smem > 64 * 1024)
+    OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
+  dim3 grid(static_cast<unsigned>((g.N + 16 * NB - 1) / (16 * NB)), static_cast<unsigned>((g.M + 16 * MB - 1) / (16 * MB)),
+            static_cast<unsigned>(g.batches));
+  omx_launch_timed(ctx, kernel, grid, dim3(SKINNY_WAVES * 64), smem, ctx->timing_start, ctx->timing_stop, g);
+  OMX_LAUNCH_CHECK(ctx, "gemm_skinny_kernel");
+  return OMX_OK;
+}
+
+}  // namespace
+
+bool omx_gemm_skinny_eligible(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km) {
+  if (a_km || b_km || g.K % 32 != 0 || !g.a_vec || !g.b_vec) return false;
+  return skinny_tile(g, ctx->cu_count > 0 ? ctx->cu_count : 256) >= 0;
+}
+
+int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g) {
+  switch (skinny_tile(g, ctx->cu_count > 0 ? ctx->cu_count : 256)) {
+    case 0: return launch_skinny<1, 1>(ctx, g);
+    case 1: return launch_skinny<1, 2>(ctx, g);
+    case 2: return launch_skinny<2, 2>(ctx, g);
+    default: return launch_skinny<4, 4>(ctx, g);
+  }
+}

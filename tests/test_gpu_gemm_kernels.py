@@ -348,3 +348,31 @@ def test_strided_batch_refuses_bad_strides(be):
         be.gemm_strided_batch(a, (1, 64), b, (64, 1), 64, 64, 64, 2, (64 * 64 + 2, 64 * 64, 64 * 64))
     with pytest.raises(OjasError):  # overlapping outputs
         be.gemm_strided_batch(a, (1, 64), b, (64, 1), 64, 64, 64, 2, (64 * 64, 64 * 64, 64))
+
+
+@pytest.mark.parametrize("rows,k,n", [(1, 32, 1), (1, 768, 770), (3, 96, 17), (16, 2048, 33), (17, 320, 64), (31, 64, 5001),
+                                      (32, 1312, 31), (65, 256, 300), (200, 768, 768), (1000, 224, 900)])
+def test_few_rows_share_k_between_waves(be, rows, k, n):
+    """gemm_skinny_kernel: every tile of its rule, rows and columns off the 16-block grid, steps that its eight
+    waves share unevenly or not at all; f32 and bf16 outputs, accumulation, the activation's store pass."""
+    from ojas_amd.backend import BF16
+
+    print(f"skinny {rows}x{k}x{n}", flush=True)
+    be.set_option("gemm_dma", 1)
+    r = orc.SplitMix64(9100 + rows + n)
+    x = orc.round_bf16(r.vec(rows * k, 0.5)).reshape(rows, k)
+    w = orc.round_bf16(r.vec(n * k, 0.5)).reshape(n, k)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = max(1.0, float(np.abs(want).max()))
+    dx, dw = be.upload(x, BF16), be.upload(w, BF16)
+    assert np.abs(be.download(be.linear_forward(dx, dw)) - want).max() <= 1e-5 * scale
+    assert np.abs(be.download_f32(be.linear_forward(dx, dw, out_dtype=BF16)) - want).max() <= 5e-3 * scale
+    c0 = r.vec(rows * n, 0.5).reshape(rows, n)
+    dc = be.upload(c0)
+    be.gemm(dx, (k, 1), dw, (1, k), rows, k, n, c=dc)
+    assert np.abs(be.download(dc) - (want + c0)).max() <= 1e-5 * scale
+    u, act = be.linear_gelu_forward(dx, dw)
+    hu = be.download_f32(u)
+    assert np.abs(hu - want).max() <= 5e-3 * scale
+    ref = orc.gelu_erf_forward(hu.reshape(-1)).reshape(rows, n)
+    assert np.abs(be.download_f32(act) - ref).max() <= 1e-2 * max(1.0, float(np.abs(ref).max()))
