@@ -496,35 +496,66 @@ __device__ __forceinline__ bool ranks_before(float va, unsigned int ia, float vb
   return ka > kb || (ka == kb && ia < ib);
 }
 
-__global__ void argmax_rows_kernel(const float* __restrict__ x, size_t rows, unsigned int cols,
-                                   unsigned int* __restrict__ out, OmxFaultWord* fault, unsigned long long tag) {
-  const int lane = threadIdx.x & 63;
-  const size_t row = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
+// One workgroup per row. The row is read once, in 16-byte pieces between its first and last aligned element;
+// what bounds it is latency, so a long row takes 1024 threads with eight pieces in flight each (one wave per row
+// walked 50304 columns in 786 dependent loads: 209 us for one row, now 10). Ties go to the lowest
+// column: every comparison prefers it, so the order in which threads meet does not matter.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void argmax_rows_kernel(const float* __restrict__ x, unsigned int cols,
+                                                              unsigned int* __restrict__ out, OmxFaultWord* fault,
+                                                              unsigned long long tag) {
+  __shared__ float wave_best[THREADS / 64];
+  __shared__ unsigned int wave_idx[THREADS / 64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const size_t row = blockIdx.x;
   const float* r = x + row * cols;
-  // Ties go to the lowest column: strict > within a lane's ascending walk.
   float best = -INFINITY;
   unsigned int idx = 0xffffffffu;
   bool bad = false;
-  for (unsigned int c = lane; c < cols; c += 64) {
-    float v = r[c];
+  auto take = [&](float v, unsigned int c) {
     bad |= !dev_finite(v);
-    if (idx == 0xffffffffu || v > best) {
+    if (idx == 0xffffffffu || v > best || (v == best && c < idx)) {
       best = v;
       idx = c;
     }
-  }
+  };
+  const unsigned int lead = min(cols, static_cast<unsigned int>((16 - (reinterpret_cast<uintptr_t>(r) & 15)) & 15) / 4);
+  const unsigned int pieces = (cols - lead) / 4;
+  if (tid < static_cast<int>(lead)) take(r[tid], tid);
+  const float4* body = reinterpret_cast<const float4*>(r + lead);
+  for (unsigned int p0 = tid; p0 < pieces; p0 += 8 * THREADS) {
+    float4 v[8];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    float ov = __shfl_xor(best, off, 64);
-    unsigned int oi = __shfl_xor(idx, off, 64);
+    for (int i = 0; i < 8; ++i) v[i] = body[min(p0 + i * THREADS, pieces - 1)];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const unsigned int c = lead + min(p0 + i * THREADS, pieces - 1) * 4;  // a repeated piece changes nothing
+      take(v[i].x, c);
+      take(v[i].y, c + 1);
+      take(v[i].z, c + 2);
+      take(v[i].w, c + 3);
+    }
+  }
+  for (unsigned int c = lead + pieces * 4 + tid; c < cols; c += THREADS) take(r[c], c);
+  auto meet = [&](float ov, unsigned int oi) {
     if (oi != 0xffffffffu && (idx == 0xffffffffu || ov > best || (ov == best && oi < idx))) {
       best = ov;
       idx = oi;
     }
+  };
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float ov = __shfl_xor(best, off, 64);
+    const unsigned int oi = __shfl_xor(idx, off, 64);
+    meet(ov, oi);
   }
-  bad = __any(bad);
   if (lane == 0) {
+    wave_best[tid >> 6] = best;
+    wave_idx[tid >> 6] = idx;
+  }
+  bad = __syncthreads_or(bad);
+  if (tid == 0) {
+    for (int w = 1; w < THREADS / 64; ++w) meet(wave_best[w], wave_idx[w]);
     out[row] = idx;
     if (bad) dev_raise_fault(fault, tag);
   }
@@ -881,9 +912,15 @@ int32_t omx_argmax_rows(omx_ctx* ctx, const void* x, uint64_t rows, uint64_t col
   if (!x || !out) return omx_fail(ctx, OMX_PLACEMENT, "argmax_rows: null device pointer");
   if (rows == 0 || cols == 0) return omx_fail(ctx, OMX_SHAPE, "argmax_rows: zero-sized axis");
   if (cols > 0xfffffffeull) return omx_fail(ctx, OMX_OUT_OF_RANGE, "argmax_rows: cols does not fit in u32");
-  hipLaunchKernelGGL(argmax_rows_kernel, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(ROW_THREADS), 0,
-                     ctx->stream, static_cast<const float*>(x), rows, static_cast<unsigned int>(cols),
-                     static_cast<unsigned int*>(out), ctx->fault, omx_tag(ctx, F_ARGMAX));
+  if (rows > 0x7fffffffull) return omx_fail(ctx, OMX_OUT_OF_RANGE, "argmax_rows: rows does not fit in i32");
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(threads), 0, ctx->stream, static_cast<const float*>(x),
+                       static_cast<unsigned int>(cols), static_cast<unsigned int*>(out), ctx->fault, omx_tag(ctx, F_ARGMAX));
+  };
+  // A quarter of a thousand columns feeds a wave; from four thousand on a row has work for sixteen.
+  if (cols <= 256) launch(&argmax_rows_kernel<64>, 64);
+  else if (cols <= 4096) launch(&argmax_rows_kernel<256>, 256);
+  else launch(&argmax_rows_kernel<1024>, 1024);
   OMX_LAUNCH_CHECK(ctx, "argmax_rows_kernel");
   return OMX_OK;
 }

@@ -848,3 +848,12 @@ def test_causal_sdpa_backward_reads_out_and_grad_output_in_their_own_dtypes(be, 
     for a, c2, og in zip(one, two, (ogq, ogk, ogv)):
         assert np.array_equal(be.download(a), be.download(c2))
         close(be.download(a), og, F32_TOL, "f32 recompute")
+
+
+@pytest.mark.parametrize("cols", [1, 3, 64, 255, 257, 4096, 4099, 50257])
+def test_argmax_of_rows_at_every_alignment(be, cols):
+    """Rows that start off a 16-byte boundary, each workgroup size, a tie that the lowest column wins."""
+    x = np.random.default_rng(cols).standard_normal((5, cols)).astype(np.float32)
+    x[1, :] = -7.0
+    x[2, [cols // 3, cols - 1]] = 9.0
+    assert np.array_equal(be.download(be.argmax_rows(be.upload(x))), np.argmax(x, axis=1).astype(np.uint32))
