@@ -105,12 +105,18 @@ int32_t omx_open(int32_t device, uint64_t budget_bytes, omx_ctx** out) {
     delete ctx;
     return OMX_UNSUPPORTED;
   }
-  if (hipStreamCreate(&ctx->stream) != hipSuccess || hipMalloc(&ctx->fault, sizeof(OmxFaultWord)) != hipSuccess ||
+  if (hipStreamCreate(&ctx->stream) != hipSuccess || hipMalloc(&ctx->fault, 256) != hipSuccess ||
       hipHostMalloc(&ctx->fault_host, sizeof(OmxFaultWord)) != hipSuccess) {
     delete ctx;
     return OMX_BACKEND;
   }
   if (reset_fault(ctx) != OMX_OK) {
+    delete ctx;
+    return OMX_BACKEND;
+  }
+  static_assert(sizeof(OmxFaultWord) <= 64, "the refused-write word lies behind the fault word");
+  ctx->kv_refused = reinterpret_cast<unsigned int*>(reinterpret_cast<char*>(ctx->fault) + 64);
+  if (omx_fill_zero(ctx, ctx->kv_refused, 64) != OMX_OK || hipStreamSynchronize(ctx->stream) != hipSuccess) {
     delete ctx;
     return OMX_BACKEND;
   }

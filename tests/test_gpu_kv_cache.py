@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import oracle_api as orc
+from ojas_amd.backend import BF16, OjasError
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
@@ -146,3 +147,40 @@ def test_refusals_and_the_deferred_fault(be):
     with pytest.raises(OjasError) as e:
         be.sync()
     assert e.value.code == NON_FINITE and "cached_attention_forward" in str(e.value)
+
+
+@pytest.mark.parametrize("batch,tn,heads,d,capacity,at", [
+    (1, 1, 1, 3, 5, 4), (64, 1, 4, 64, 40, 39), (64, 1, 12, 64, 40, 39), (3, 37, 4, 64, 50, 30), (2, 90, 6, 64, 90, 77), (5, 70, 7, 31, 100, 1095)])
+@pytest.mark.parametrize("bf16_cache", [False, True])
+def test_cache_write_short_and_long(be, batch, tn, heads, d, capacity, at, bf16_cache):
+    """Both forms of the write (one launch up to 16384 values, a scan and a copy above), vector and scalar, over the
+    ring's end; a refused write leaves the cache as it is and does not hold up the next one."""
+    r = np.random.default_rng(batch * 1000 + tn)
+    old = r.standard_normal((batch, capacity, heads, d)).astype(np.float32)
+    src = r.standard_normal((batch, tn, heads, d)).astype(np.float32)
+    cache = be.upload(old, BF16) if bf16_cache else be.upload(old)
+    before = be.download(cache)
+    bad = src.copy()
+    bad.reshape(-1)[-1] = np.inf
+    be.kv_cache_write(cache, be.upload(bad), at)
+    with pytest.raises(OjasError):
+        be.sync()
+    assert np.array_equal(be.download(cache), before)
+    be.kv_cache_write(cache, be.upload(src), at)
+    want = before.copy()
+    values = be.download(be.upload(src, BF16)) if bf16_cache else src
+    for j in range(tn):
+        want[:, (at + j) % capacity] = values[:, j]
+    assert np.array_equal(be.download(cache), want)
+
+
+@pytest.mark.parametrize("b,tq,h,hkv,d,kv_len", [
+    (1, 1, 1, 1, 64, 1), (1, 1, 12, 12, 64, 301), (2, 1, 12, 4, 128, 700), (70, 1, 8, 8, 64, 129), (130, 1, 8, 8, 32, 67),
+    (1, 1, 2, 2, 64, 4500)])
+def test_decode_rows_under_every_block_shape(be, b, tq, h, hkv, d, kv_len):
+    """Eight, four and one wave per block; one part (written by the block itself) and several (merged)."""
+    r = np.random.default_rng(kv_len)
+    q, k, v = (r.standard_normal(s).astype(np.float32) for s in ((b, tq, h, d), (b, kv_len, hkv, d), (b, kv_len, hkv, d)))
+    want = orc.cached_attention_forward(q, k, v, kv_len)
+    got = be.download(be.cached_attention_forward(be.upload(q), be.upload(k), be.upload(v), kv_len))
+    assert np.abs(got - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))
