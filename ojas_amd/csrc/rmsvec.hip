@@ -18,62 +18,6 @@ namespace {
 
 constexpr int RV_THREADS = 256;
 
-template <typename TX, typename TA, typename TY, int NCH>
-__global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __restrict__ x, const TA* __restrict__ add,
-                                                                 const float* __restrict__ w,
-                                                                 float* __restrict__ sum_out, TY* __restrict__ y,
-                                                                 size_t rows, int dim, float eps, OmxFaultWord* fault,
-                                                                 unsigned long long tag) {
-  const int lane = threadIdx.x & 63;
-  const size_t row = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const size_t base = row * dim;
-  float xv[NCH][4];
-  float ss = 0.0f;
-  bool bad = false;
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int c = j * 256 + lane * 4;
-    if (c < dim) {
-      dev_load4<TX>(x, base + c, xv[j]);
-      if (add) {
-        float av[4];
-        dev_load4<TA>(add, base + c, av);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          xv[j][e] = xv[j][e] + av[e];
-          bad |= !dev_finite(xv[j][e]);
-        }
-        dev_store4<float>(sum_out, base + c, xv[j]);
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) xv[j][e] = 0.0f;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss += xv[j][e] * xv[j][e];
-  }
-  ss = wave_sum(ss);
-  const float denom = ss / static_cast<float>(dim) + eps;
-  const float rstd = 1.0f / sqrtf(denom);
-  bad |= !(dev_finite(denom) && denom > 0.0f && dev_finite(rstd));
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int c = j * 256 + lane * 4;
-    if (c < dim) {
-      float wv[4], out[4];
-      dev_load4<float>(w, c, wv);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        out[e] = xv[j][e] * rstd * wv[e];
-        bad |= !dev_finite(out[e]);
-      }
-      dev_store4<TY>(y, base + c, out);
-    }
-  }
-  if (bad) dev_raise_fault(fault, tag);
-}
-
 // Four elements as they sit in memory: the row waits in registers in this form between the passes
 // (a bf16 operand at half the registers of its f32 values).
 template <typename T>
@@ -93,6 +37,76 @@ struct Raw4<unsigned short> {
     v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
   }
 };
+
+// All of a row's loads (the weight row too, up to 1024 columns) are issued before the first is used: with the
+// sum stored between one chunk's loads and the next chunk's, a row was NCH + 1 memory latencies in a chain,
+// which is all there is to a call of a few rows (1024 rows of 768: 6.5 -> 4.5 us with the launch).
+template <typename TX, typename TA, typename TY, int NCH>
+__global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __restrict__ x, const TA* __restrict__ add,
+                                                                 const float* __restrict__ w,
+                                                                 float* __restrict__ sum_out, TY* __restrict__ y,
+                                                                 size_t rows, int dim, float eps, OmxFaultWord* fault,
+                                                                 unsigned long long tag) {
+  constexpr bool EARLY_W = NCH <= 4;
+  const int lane = threadIdx.x & 63;
+  const size_t row = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const size_t base = row * dim;
+  Raw4<TX> xr[NCH];
+  Raw4<TA> ar[NCH];
+  Raw4<float> wr[EARLY_W ? NCH : 1];
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    const int c = j * 256 + lane * 4;
+    if (c < dim) {
+      xr[j].load(x + base + c);
+      if (add) ar[j].load(add + base + c);
+      if constexpr (EARLY_W) wr[j].load(w + c);
+    } else {
+      xr[j].clear();
+      ar[j].clear();
+    }
+  }
+  float xv[NCH][4];
+  float ss = 0.0f;
+  bool bad = false;
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    xr[j].get(xv[j]);
+    if (add) {
+      float av[4];
+      ar[j].get(av);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xv[j][e] = xv[j][e] + av[e];
+        bad |= !dev_finite(xv[j][e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += xv[j][e] * xv[j][e];
+  }
+  ss = wave_sum(ss);
+  const float denom = ss / static_cast<float>(dim) + eps;
+  const float rstd = 1.0f / sqrtf(denom);
+  bad |= !(dev_finite(denom) && denom > 0.0f && dev_finite(rstd));
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    const int c = j * 256 + lane * 4;
+    if (c < dim) {
+      float wv[4], out[4];
+      if constexpr (EARLY_W) wr[j].get(wv);
+      else dev_load4<float>(w, c, wv);
+      if (add) dev_store4<float>(sum_out, base + c, xv[j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        out[e] = xv[j][e] * rstd * wv[e];
+        bad |= !dev_finite(out[e]);
+      }
+      dev_store4<TY>(y, base + c, out);
+    }
+  }
+  if (bad) dev_raise_fault(fault, tag);
+}
 
 // gx = rms_norm_backward(x, w, gy) (+ add_in), optionally also stored as bf16;
 // per-block partial column sums of gy * xhat for the weight gradient.
