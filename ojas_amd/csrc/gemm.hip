@@ -476,6 +476,10 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   // Few rows (a decoder's linear layers): K shared between a workgroup's waves, no tile of 128 rows.
   const bool skinny = operand_dtype == OMX_BF16 && !thin && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0 &&
                       omx_gemm_skinny_eligible(ctx, g, a_km, b_km);
+  // f32 outputs of less than a few rounds of 128 x 128 tiles.
+  int frag32 = -1;
+  if (operand_dtype == OMX_F32 && ctx->gemm_dma_mode == 1 && !(epi && epi->mode != OMX_EPI_NONE))
+    frag32 = omx_gemm_frag32_tile(ctx, g, a_km, b_km);
   int dma_variant = -1;
   if (!thin && !skinny && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km)) {
     const int mode = ctx->gemm_dma_mode;
@@ -607,7 +611,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     // 108 tiles: two splits; of 2304 x 768, 324 tiles: two splits make three rounds of half the length).
     const long all_tiles = tiles * g.batches;
     const bool may_split =
-        !thin && !skinny && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
+        !thin && !skinny && frag32 < 0 && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
     if (may_split && ksteps >= 4 * min_steps && !(epi && epi->mode != OMX_EPI_NONE)) {
       splits = static_cast<int>(((g.batches == 1 ? 512 : 1024) + all_tiles - 1) / all_tiles);
       if (splits > ksteps / min_steps) splits = ksteps / min_steps;
@@ -679,6 +683,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   int32_t rc;
   if (thin) {
     rc = omx_gemm_thin_launch(ctx, g, b_km);
+  } else if (frag32 >= 0) {
+    rc = omx_gemm_frag32_launch(ctx, g, a_km, b_km, frag32);
   } else if (skinny) {
     rc = omx_gemm_skinny_launch(ctx, g);
   } else if (dma_variant >= 0) {

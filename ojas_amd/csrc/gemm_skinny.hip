@@ -79,11 +79,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(GemmArgs g) {
   bool bad = false;
   for (int blk = wave; blk < MB * NB; blk += WAVES) {
     const int row = row0 + blk / NB * 16 + l16, col = col0 + blk % NB * 16 + (lane >> 4) * 4;
-    float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // Neighbours first: the error of a sum of eight grows with three additions, not with seven.
+    float x[4];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w)
+    for (int v = 0; v < 4; ++v) {
+      float part[WAVES];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) x[v] += skinny_red[((w * (MB * NB) + blk) * 4 + v) * 64 + lane];
+      for (int w = 0; w < WAVES; ++w) part[w] = skinny_red[((w * (MB * NB) + blk) * 4 + v) * 64 + lane];
+#pragma unroll
+      for (int span = 1; span < WAVES; span *= 2)
+#pragma unroll
+        for (int w = 0; w < WAVES; w += 2 * span) part[w] += part[w + span];
+      x[v] = part[0];
+    }
     if (row < g.M && col < g.N)
       bad |= g.epi == OMX_EPI_NONE ? gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3])
                                    : gemm_store4_epi(g, 0, row, col, x[0], x[1], x[2], x[3]);
@@ -95,7 +103,7 @@ struct SkinnyTile {
   int mb, nb;
 };
 constexpr SkinnyTile SKINNY_TILES[] = {{1, 1}, {1, 2}, {2, 2}, {4, 4}};
-constexpr int SKINNY_WAVES = 8, SKINNY_CHUNK = 4;
+constexpr int SKINNY_CHUNK = 4;
 
 // The smallest tile that makes at most one workgroup per compute unit: a workgroup's time is its own
 // operand rows (2.5 us + about 1 ns per column of K and 16-row block: a CU fetches 64-byte row pieces at
@@ -119,17 +127,22 @@ int skinny_tile(const GemmArgs& g, long units) {
   return -1;
 }
 
-template <int MB, int NB>
-int32_t launch_skinny(omx_ctx* ctx, const GemmArgs& g) {
-  constexpr int smem = SKINNY_WAVES * MB * NB * 1024;
-  auto kernel = &gemm_skinny_kernel<MB, NB, SKINNY_WAVES, SKINNY_CHUNK>;
+template <int MB, int NB, int WAVES>
+int32_t launch_skinny_waves(omx_ctx* ctx, const GemmArgs& g) {
+  constexpr int smem = WAVES * MB * NB * 1024;
+  auto kernel = &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK>;
   if constexpr (smem > 64 * 1024)
     OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
   dim3 grid(static_cast<unsigned>((g.N + 16 * NB - 1) / (16 * NB)), static_cast<unsigned>((g.M + 16 * MB - 1) / (16 * MB)),
             static_cast<unsigned>(g.batches));
-  omx_launch_timed(ctx, kernel, grid, dim3(SKINNY_WAVES * 64), smem, ctx->timing_start, ctx->timing_stop, g);
+  omx_launch_timed(ctx, kernel, grid, dim3(WAVES * 64), smem, ctx->timing_start, ctx->timing_stop, g);
   OMX_LAUNCH_CHECK(ctx, "gemm_skinny_kernel");
   return OMX_OK;
+}
+// Eight waves share K; up to 512 columns four do (two to four steps each), with half the sums to meet.
+template <int MB, int NB>
+int32_t launch_skinny(omx_ctx* ctx, const GemmArgs& g) {
+  return g.K <= 512 ? launch_skinny_waves<MB, NB, 4>(ctx, g) : launch_skinny_waves<MB, NB, 8>(ctx, g);
 }
 
 }  // namespace

@@ -376,3 +376,29 @@ def test_few_rows_share_k_between_waves(be, rows, k, n):
     assert np.abs(hu - want).max() <= 5e-3 * scale
     ref = orc.gelu_erf_forward(hu.reshape(-1)).reshape(rows, n)
     assert np.abs(be.download_f32(act) - ref).max() <= 1e-2 * max(1.0, float(np.abs(ref).max()))
+
+
+@pytest.mark.parametrize("rows,k,n", [(16, 16, 16), (16, 4, 16), (48, 20, 32), (100, 260, 36), (256, 256, 256), (130, 8, 62), (704, 256, 704),
+                                      (1030, 72, 260), (52, 3000, 44), (2048, 256, 256), (31, 64, 29)])
+def test_small_f32_outputs_share_k_between_waves(be, rows, k, n):
+    """gemm_frag32_kernel: the tiles of its rule in all operand layouts, rows and columns off the tile, K off the
+    16-column step (and shorter than one), more waves than steps, accumulation and a strided batch."""
+    print(f"frag32 {rows}x{k}x{n}", flush=True)
+    be.set_option("gemm_dma", 1)
+    r = orc.SplitMix64(7700 + rows + n)
+    a, b, c0 = (r.vec(x * y, 0.5).reshape(x, y) for x, y in ((rows, k), (k, n), (rows, n)))
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    tol = 1e-5 * max(1.0, float(np.abs(want).max()))
+    da, dat, db, dbt = (be.upload(np.ascontiguousarray(x)) for x in (a, a.T, b, b.T))
+    for x, xs in ((da, (k, 1)), (dat, (1, rows))):
+        for y, ys in ((db, (n, 1)), (dbt, (1, k))):
+            got = be.download(be.gemm(x, xs, y, ys, rows, k, n))
+            assert np.abs(got - want).max() <= tol, (xs, ys)
+            c = be.upload(c0)
+            be.gemm(x, xs, y, ys, rows, k, n, c=c)
+            assert np.abs(be.download(c) - (want + c0)).max() <= tol, (xs, ys)
+    if rows * k % 4 == 0 and k * n % 4 == 0 and rows * n % 4 == 0:
+        many = be.gemm_strided_batch(be.upload(np.stack([a, -a, 2 * a])), (k, 1), be.upload(np.stack([b, b, b])), (n, 1), rows, k, n, 3,
+                                     (rows * k, k * n, rows * n))
+        got = be.download(many).reshape(3, rows, n)
+        assert np.abs(got - np.stack([want, -want, 2 * want])).max() <= 2 * tol
