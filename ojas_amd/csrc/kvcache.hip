@@ -22,6 +22,7 @@
 #include <algorithm>
 
 #include "omx_common.h"
+#include "sdpa_mfma32.h"
 
 namespace {
 
@@ -618,6 +619,37 @@ int32_t omx_cached_attention_forward(omx_ctx* ctx, const void* q, const void* k_
   const uint64_t rows_total = batch * tq * heads;
   if (batch * kv_heads > 65535 || rows_total > 0x7fffffffull || capacity > 0x7fffffffull || kv_len > (1ull << 40))
     return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: extent too large", op);
+
+  // A prompt chunk: from 16 rows per KV head on, every tile of keys serves 16 rows and more, and the products go to
+  // the matrix units (the kernels below read a key's row once per 4 or 8 query rows and take the sums on vector
+  // instructions). 4 x 12 heads, 256 new positions of 700: 186 -> 38 us per call.
+  const bool bf16 = cache_dtype == OMX_BF16;
+  const long step = static_cast<long>(kv_heads * head_dim);
+  if (tq * (heads / kv_heads) >= 16 && tq * (heads / kv_heads) <= 0x7fffffffull && ctx->kv_attention_mode == 0 &&
+      omx_sdpa32_supports(head_dim, batch * kv_heads, {q, k_cache, v_cache, out}, {})) {
+    Sdpa32Args m{};
+    m.q = static_cast<const float*>(q);
+    m.k = k_cache;
+    m.v = v_cache;
+    m.out = static_cast<float*>(out);
+    m.q_h = m.o_h = m.k_h = static_cast<long>(head_dim);
+    m.q_t = m.o_t = static_cast<long>(heads * head_dim);
+    m.q_b = m.o_b = static_cast<long>(tq * heads * head_dim);
+    m.k_t = step;
+    m.k_b = static_cast<long>(capacity) * step;
+    m.kv_heads = static_cast<int>(kv_heads);
+    m.rep = static_cast<int>(heads / kv_heads);
+    m.tq = static_cast<int>(tq);
+    m.tk = static_cast<int>(span);
+    m.q_pos0 = static_cast<int>(span - tq);
+    m.slot0 = static_cast<int>((kv_len - span) % capacity);
+    m.capacity = static_cast<int>(capacity);
+    m.window = window < span ? static_cast<int>(window) : 0;
+    m.scale = 1.0f / std::sqrt(static_cast<float>(head_dim));
+    m.fault = ctx->fault;
+    m.tag = omx_tag(ctx, F_CACHED_ATTENTION);
+    return omx_sdpa32_forward(ctx, m, static_cast<int>(batch), static_cast<int>(head_dim), bf16);
+  }
 
   KvArgs a;
   a.q = static_cast<const float*>(q);

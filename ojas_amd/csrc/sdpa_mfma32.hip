@@ -1,0 +1,640 @@
+// f32 attention on the f32 matrix instructions (v_mfma_f32_16x16x4_f32), head dims 16 / 32 / 64 / 128: causal SDPA
+// forward and backward of the f32 tier and the attention of a prompt chunk over a KV cache.
+//
+// Reference: ojas-cpu/src/attn.rs (causal_sdpa_*; trait ojas-core/src/backend.rs:1729-1792) and
+// ojas-cpu/src/kv.rs (cached_attention_forward, backend.rs:2526-2555). Same formulas as sdpa.hip's row
+// kernels: p = e^(s - max), out = sum p v / sum p, lse = max + ln(sum); backward p = e^(s - lse),
+// dS = scale p (dP - dO . O).
+//
+// What bounds it: the matrix units have the vector units' f32 rate (157 TFLOP/s) but take their operands from a
+// quarter of the LDS traffic. On vector instructions 64 x 64 tiles ran at 5 to 12 % of that rate, bound by LDS reads,
+// and the key / value pass of a grouped model had a workgroup per 64 keys of a KV head: 52 for 256 units.
+//
+// Rows are packed: row r of a KV head is query r / rep of its head r % rep, so grouped heads share every key
+// and value tile. Score tiles are formed with the rows that softmax runs over in the accumulator's registers (lane
+// l: row l % 16, values 4 (l / 16) + v), which is exactly the operand layout of the product that follows (its
+// instruction j takes K values 4 (l / 16) + j): probabilities and dS go from accumulator to operand without
+// moving. The other operand of that product is read from LDS along its fast index: one 16-byte read serves four
+// interleaved blocks of result columns (block c VW + e holds columns 16 VW c + VW i + e).
+//
+// 64-row tiles are fetched into registers while the previous one is multiplied. Where there are few rows the four
+// waves of a workgroup split the keys (KW = 4) instead of the rows and meet in LDS; the key / value pass splits
+// its rows over the grid when keys alone do not fill the chip, and a second launch adds the parts in order.
+// No atomics; every sum has a fixed order.
+//
+// Before and after, us, forward / backward (batch x heads over KV heads x time x head dim): 8 x 4/4 x 256 x 64: 38 / 109 ->
+// 13 / 34; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370 -> 20 / 66; 16 x 12/12 x 512 x 64: 272 / 1337 -> 132 / 439 (48 and
+// 37 TFLOP/s, causal-counted); 1 x 2/1 x 3000 x 128: 696 / 3334 -> 151 / 409.
+#include <algorithm>
+#include <cmath>
+
+#include "sdpa_mfma32.h"
+
+namespace {
+
+typedef float floatx4_a __attribute__((ext_vector_type(4)));
+constexpr int AT_THREADS = 256, AT_ROWS = 64;  // rows per LDS tile
+constexpr float AT_LOG2E = 1.4426950408889634f, AT_LN2 = 0.6931471805599453f;
+
+__device__ __forceinline__ floatx4_a at_mfma(float a, float b, floatx4_a c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ floatx4_a at_zero() { return floatx4_a{0.0f, 0.0f, 0.0f, 0.0f}; }
+// Over the four lanes that hold one row.
+__device__ __forceinline__ float at_row_max(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16));
+  return fmaxf(v, __shfl_xor(v, 32));
+}
+__device__ __forceinline__ float at_row_sum(float v) {
+  v += __shfl_xor(v, 16);
+  return v + __shfl_xor(v, 32);
+}
+
+template <int D>
+struct AtDim {
+  static constexpr int S = D / 16;             // 16-column steps of a product over the head dim; column blocks of a result
+  static constexpr int VW = S < 4 ? S : 4;     // interleaved column blocks per LDS read
+  static constexpr int NC = S / VW;
+  static constexpr int P = D + 4;              // LDS row pitch: 16 rows' 16-byte pieces fall in distinct banks
+  static constexpr int PIECES = AT_ROWS * D / 4 / AT_THREADS;  // 16-byte pieces of a tile per thread (at least 1)
+};
+
+// A tile on its way: PIECES pieces per thread, in memory's type until they are stored.
+template <int D, typename T>
+struct AtTile {
+  using Raw = std::conditional_t<sizeof(T) == 4, float4, uint2>;
+  Raw raw[AtDim<D>::PIECES];
+  // `row_at(r)`: pointer to tile row r, or null for a row of zeros.
+  template <typename F>
+  __device__ __forceinline__ void fetch(F row_at) {
+#pragma unroll
+    for (int i = 0; i < AtDim<D>::PIECES; ++i) {
+      const int idx = threadIdx.x + i * AT_THREADS, r = idx / (D / 4), c = idx % (D / 4);
+      const T* p = row_at(r);
+      if (p) raw[i] = *reinterpret_cast<const Raw*>(p + 4 * c);
+      else raw[i] = Raw{};
+    }
+  }
+  __device__ __forceinline__ void store(float* lds) const {
+#pragma unroll
+    for (int i = 0; i < AtDim<D>::PIECES; ++i) {
+      const int idx = threadIdx.x + i * AT_THREADS, r = idx / (D / 4), c = idx % (D / 4);
+      float4 v;
+      if constexpr (sizeof(T) == 4) {
+        v = raw[i];
+      } else {
+        v = make_float4(__uint_as_float(raw[i].x << 16), __uint_as_float(raw[i].x & 0xffff0000u), __uint_as_float(raw[i].y << 16),
+                        __uint_as_float(raw[i].y & 0xffff0000u));
+      }
+      *reinterpret_cast<float4*>(lds + r * AtDim<D>::P + 4 * c) = v;
+    }
+  }
+};
+
+// acc (values 4 g + v of 16 tile rows, this lane's own row) = tile rows . own row over the head dim.
+template <int D>
+__device__ __forceinline__ floatx4_a at_dot(const float* tile16, const float4 (&own)[AtDim<D>::S], int i, int g) {
+  floatx4_a acc = at_zero();
+  const float* p = tile16 + i * AtDim<D>::P + 4 * g;
+#pragma unroll
+  for (int s = 0; s < AtDim<D>::S; ++s) {
+    const float4 t = *reinterpret_cast<const float4*>(p + 16 * s);
+    acc = at_mfma(t.x, own[s].x, acc);
+    acc = at_mfma(t.y, own[s].y, acc);
+    acc = at_mfma(t.z, own[s].z, acc);
+    acc = at_mfma(t.w, own[s].w, acc);
+  }
+  return acc;
+}
+// out[block] += sum over 16 tile rows of weight[row] * tile row, weights in at_dot's layout.
+template <int D>
+__device__ __forceinline__ void at_accumulate(const float* tile16, const floatx4_a& weight, floatx4_a (&out)[AtDim<D>::S], int i, int g) {
+  using X = AtDim<D>;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float* row = tile16 + (4 * g + j) * X::P + X::VW * i;
+#pragma unroll
+    for (int c = 0; c < X::NC; ++c) {
+      float t[X::VW];
+      if constexpr (X::VW == 4) {
+        const float4 x = *reinterpret_cast<const float4*>(row + 64 * c);
+        t[0] = x.x; t[1] = x.y; t[2] = x.z; t[3] = x.w;
+      } else if constexpr (X::VW == 2) {
+        const float2 x = *reinterpret_cast<const float2*>(row);
+        t[0] = x.x; t[1] = x.y;
+      } else {
+        t[0] = *row;
+      }
+#pragma unroll
+      for (int e = 0; e < X::VW; ++e) out[c * X::VW + e] = at_mfma(t[e], weight[j], out[c * X::VW + e]);
+    }
+  }
+}
+// A row's result columns held by this lane, times `f`, for accumulator registers v0 .. v0 + NV - 1.
+template <int D, int NV>
+__device__ __forceinline__ bool at_store(float* row, const floatx4_a (&out)[AtDim<D>::S], float f, int g, int v0) {
+  using X = AtDim<D>;
+  bool bad = false;
+#pragma unroll
+  for (int c = 0; c < X::NC; ++c)
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      float* p = row + c * 16 * X::VW + X::VW * (4 * g + v0 + u);
+#pragma unroll
+      for (int e = 0; e < X::VW; ++e) {
+        float x = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x = v == v0 + u ? out[c * X::VW + e][v] : x;  // a register index known only when NV < 4
+        x *= f;
+        bad |= !dev_finite(x);
+        p[e] = x;
+      }
+    }
+  return bad;
+}
+
+struct AtRow {
+  int query, head;  // head within the group
+};
+__device__ __forceinline__ AtRow at_unpack(int r, int rep) {
+  AtRow x;
+  if (rep == 1) {
+    x.query = r;
+    x.head = 0;
+  } else {
+    x.query = r / rep;
+    x.head = r - x.query * rep;
+  }
+  return x;
+}
+// Own row `r` of a [.., row, D] tensor as a product operand.
+template <int D>
+__device__ __forceinline__ void at_own(const float* row, float4 (&own)[AtDim<D>::S], int g) {
+#pragma unroll
+  for (int s = 0; s < AtDim<D>::S; ++s) own[s] = *reinterpret_cast<const float4*>(row + 16 * s + 4 * g);
+}
+
+// ---------------------------------------------------------------- forward
+template <int D, int KW, typename TK>
+__global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
+  using X = AtDim<D>;
+  constexpr int QW = 4 / KW, BQ = 16 * QW, NB = AT_ROWS / 16 / KW;
+  __shared__ __align__(16) float lds[2 * AT_ROWS * X::P];
+  float* kt = lds;
+  float* vt = lds + AT_ROWS * X::P;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int qw = wave % QW, kw = wave / QW;
+  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const int rows = a.tq * a.rep;
+  const int r0 = (gridDim.x - 1 - blockIdx.x) * BQ;  // the rows that see the most keys first
+  const int r = r0 + qw * 16 + i;
+  const AtRow at = at_unpack(min(r, rows - 1), a.rep);
+  const long q_at = b * a.q_b + (static_cast<long>(kvh) * a.rep + at.head) * a.q_h + static_cast<long>(at.query) * a.q_t;
+  float4 q[X::S];
+  at_own<D>(a.q + q_at, q, g);
+  const int pos = r < rows ? a.q_pos0 + at.query : -1;
+  const int low = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
+  const int first_pos = a.q_pos0 + at_unpack(r0, a.rep).query;
+  const int last_pos = a.q_pos0 + at_unpack(min(r0 + BQ, rows) - 1, a.rep).query;
+  const int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / AT_ROWS, t_last = last_pos / AT_ROWS;
+  const TK* kb = static_cast<const TK*>(a.k) + b * a.k_b + kvh * a.k_h;
+  const TK* vb = static_cast<const TK*>(a.v) + b * a.k_b + kvh * a.k_h;
+  AtTile<D, TK> kn, vn;
+  auto fetch = [&](int t) {
+    auto slot_at = [&](int row) {
+      const int key = t * AT_ROWS + row;
+      int slot = a.slot0 + key;  // a ring wraps at most once over the keys that are read
+      slot = slot >= a.capacity ? slot - a.capacity : slot;
+      return key < a.tk ? slot : -1;
+    };
+    kn.fetch([&](int row) { const int s = slot_at(row); return s < 0 ? nullptr : kb + static_cast<long>(s) * a.k_t; });
+    vn.fetch([&](int row) { const int s = slot_at(row); return s < 0 ? nullptr : vb + static_cast<long>(s) * a.k_t; });
+  };
+  const float scale2 = a.scale * AT_LOG2E;
+  floatx4_a o[X::S];
+#pragma unroll
+  for (int m = 0; m < X::S; ++m) o[m] = at_zero();
+  float mx = -INFINITY, sum = 0.0f;  // in the exp2 domain; `sum` over this lane's keys only
+  bool bad = false;
+  fetch(t_first);
+  for (int t = t_first; t <= t_last; ++t) {
+    __syncthreads();  // the previous tile has been read
+    kn.store(kt);
+    vn.store(vt);
+    __syncthreads();
+    if (t < t_last) fetch(t + 1);
+    floatx4_a s[NB];
+    float top = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const int row = (kw * NB + n) * 16;
+      s[n] = at_dot<D>(kt + row * X::P, q, i, g);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int key = t * AT_ROWS + row + 4 * g + v;
+        const bool seen = key <= pos && key >= low;
+        const float x = s[n][v] * scale2;
+        bad |= seen && !dev_finite(x);
+        s[n][v] = seen ? x : -INFINITY;
+        top = fmaxf(top, s[n][v]);
+      }
+    }
+    top = at_row_max(top);
+    const float mx_new = fmaxf(mx, top), base = mx_new == -INFINITY ? 0.0f : mx_new;
+    const float rescale = __builtin_amdgcn_exp2f(mx - base);  // 0 on the first keys; 1 when none were seen yet: the sums are 0
+    mx = mx_new;
+    sum *= rescale;
+#pragma unroll
+    for (int m = 0; m < X::S; ++m)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o[m][v] *= rescale;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        s[n][v] = __builtin_amdgcn_exp2f(s[n][v] - base);
+        sum += s[n][v];
+      }
+      at_accumulate<D>(vt + (kw * NB + n) * 16 * X::P, s[n], o, i, g);
+    }
+  }
+  sum = at_row_sum(sum);
+  float* out = a.out + b * a.o_b + (static_cast<long>(kvh) * a.rep + at.head) * a.o_h + static_cast<long>(at.query) * a.o_t;
+  float* lse = a.lse ? a.lse + (static_cast<long>(b) * a.kv_heads * a.rep + static_cast<long>(kvh) * a.rep + at.head) * a.tq + at.query : nullptr;
+  if constexpr (KW == 1) {
+    if (r < rows) {
+      bad |= !(dev_finite(sum) && sum > 0.0f);
+      bad |= at_store<D, 4>(out, o, 1.0f / sum, g, 0);
+      if (lse && g == 0) *lse = mx * AT_LN2 + logf(sum);
+    }
+  } else {
+    // The four waves' shares of the same rows: every wave adds up one register of each block.
+    __syncthreads();
+    float* stat = lds;                   // [4][2][16]
+    float* part = lds + 128;             // [4][S * 4][64]
+    if (g == 0) {
+      stat[kw * 32 + i] = mx;
+      stat[kw * 32 + 16 + i] = sum;
+    }
+#pragma unroll
+    for (int m = 0; m < X::S; ++m)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) part[((kw * X::S + m) * 4 + v) * 64 + lane] = o[m][v];
+    __syncthreads();
+    float all = -INFINITY, weight[4], total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) all = fmaxf(all, stat[w * 32 + i]);
+    const float base = all == -INFINITY ? 0.0f : all;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      weight[w] = __builtin_amdgcn_exp2f(stat[w * 32 + i] - base);
+      total = fmaf(weight[w], stat[w * 32 + 16 + i], total);
+    }
+#pragma unroll
+    for (int m = 0; m < X::S; ++m) {
+      float x = 0.0f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) x = fmaf(weight[w], part[((w * X::S + m) * 4 + kw) * 64 + lane], x);
+      o[m] = floatx4_a{x, x, x, x};
+    }
+    if (r < rows) {
+      bad |= !(dev_finite(total) && total > 0.0f);
+      bad |= at_store<D, 1>(out, o, 1.0f / total, g, kw);
+      if (lse && g == 0 && kw == 0) *lse = all * AT_LN2 + logf(total);
+    }
+  }
+  if (bad) dev_raise_fault(a.fault, a.tag);
+}
+
+// ---------------------------------------------------------------- backward
+// p and dS of one lane's four scores, from the score and dP accumulators.
+struct AtGrad {
+  float scale, scale2;
+  __device__ __forceinline__ void operator()(bool seen, float score, float dp, float lse2, float delta, float* p, float* ds,
+                                             bool* bad) const {
+    const float x = score * scale2;
+    const float pr = seen ? __builtin_amdgcn_exp2f(x - lse2) : 0.0f;
+    *bad |= seen && !(dev_finite(x) && dev_finite(pr));
+    *p = pr;
+    *ds = seen ? scale * (pr * (dp - delta)) : 0.0f;
+  }
+};
+
+// dQ, and the row term delta = dO . O when `out` is given (it is read from `delta` otherwise).
+template <int D, int KW>
+__global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
+  using X = AtDim<D>;
+  constexpr int QW = 4 / KW, BQ = 16 * QW, NB = AT_ROWS / 16 / KW;
+  __shared__ __align__(16) float lds[2 * AT_ROWS * X::P];
+  float* kt = lds;
+  float* vt = lds + AT_ROWS * X::P;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int qw = wave % QW, kw = wave / QW;
+  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const int rows = a.tq * a.rep;
+  const int r0 = (gridDim.x - 1 - blockIdx.x) * BQ;
+  const int r = r0 + qw * 16 + i;
+  const AtRow at = at_unpack(min(r, rows - 1), a.rep);
+  const long head = static_cast<long>(kvh) * a.rep + at.head;
+  const long q_at = b * a.q_b + head * a.q_h + static_cast<long>(at.query) * a.q_t;
+  const long o_at = b * a.o_b + head * a.o_h + static_cast<long>(at.query) * a.o_t;
+  float4 q[X::S], dout[X::S];
+  at_own<D>(a.q + q_at, q, g);
+  at_own<D>(a.gy + o_at, dout, g);
+  const long stat = (static_cast<long>(b) * a.kv_heads * a.rep + head) * a.tq + at.query;
+  float delta;
+  if (a.out) {
+    float4 saved[X::S];
+    at_own<D>(a.out + o_at, saved, g);
+    delta = 0.0f;
+#pragma unroll
+    for (int s = 0; s < X::S; ++s)
+      delta += dout[s].x * saved[s].x + dout[s].y * saved[s].y + dout[s].z * saved[s].z + dout[s].w * saved[s].w;
+    delta = at_row_sum(delta);
+    if (g == 0 && kw == 0 && r < rows) a.delta[stat] = delta;
+  } else {
+    delta = a.delta[stat];
+  }
+  const float lse2 = a.lse[stat] * AT_LOG2E;
+  const int pos = r < rows ? at.query : -1;
+  const int low = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
+  const int first_pos = at_unpack(r0, a.rep).query, last_pos = at_unpack(min(r0 + BQ, rows) - 1, a.rep).query;
+  const int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / AT_ROWS, t_last = last_pos / AT_ROWS;
+  const float* kb = static_cast<const float*>(a.k) + b * a.k_b + kvh * a.k_h;
+  const float* vb = static_cast<const float*>(a.v) + b * a.k_b + kvh * a.k_h;
+  AtTile<D, float> kn, vn;
+  auto fetch = [&](int t) {
+    kn.fetch([&](int row) { const int key = t * AT_ROWS + row; return key < a.tk ? kb + static_cast<long>(key) * a.k_t : nullptr; });
+    vn.fetch([&](int row) { const int key = t * AT_ROWS + row; return key < a.tk ? vb + static_cast<long>(key) * a.k_t : nullptr; });
+  };
+  const AtGrad grad{a.scale, a.scale * AT_LOG2E};
+  floatx4_a dq[X::S];
+#pragma unroll
+  for (int m = 0; m < X::S; ++m) dq[m] = at_zero();
+  bool bad = false;
+  fetch(t_first);
+  for (int t = t_first; t <= t_last; ++t) {
+    __syncthreads();
+    kn.store(kt);
+    vn.store(vt);
+    __syncthreads();
+    if (t < t_last) fetch(t + 1);
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const int row = (kw * NB + n) * 16;
+      const floatx4_a s = at_dot<D>(kt + row * X::P, q, i, g);
+      const floatx4_a dp = at_dot<D>(vt + row * X::P, dout, i, g);
+      floatx4_a ds;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int key = t * AT_ROWS + row + 4 * g + v;
+        float p, d;
+        grad(key <= pos && key >= low, s[v], dp[v], lse2, delta, &p, &d, &bad);
+        ds[v] = d;
+      }
+      at_accumulate<D>(kt + row * X::P, ds, dq, i, g);
+    }
+  }
+  float* out = a.gq + q_at;
+  if constexpr (KW == 1) {
+    if (r < rows) bad |= at_store<D, 4>(out, dq, 1.0f, g, 0);
+  } else {
+    __syncthreads();
+    float* part = lds;  // [4][S * 4][64]
+#pragma unroll
+    for (int m = 0; m < X::S; ++m)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) part[((kw * X::S + m) * 4 + v) * 64 + lane] = dq[m][v];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < X::S; ++m) {
+      float x = 0.0f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) x += part[((w * X::S + m) * 4 + kw) * 64 + lane];
+      dq[m] = floatx4_a{x, x, x, x};
+    }
+    if (r < rows) bad |= at_store<D, 1>(out, dq, 1.0f, g, kw);
+  }
+  if (bad) dev_raise_fault(a.fault, a.tag);
+}
+
+// dK and dV of 16 KG keys, over a share (blockIdx.z of gridDim.z) of the row tiles that see them.
+template <int D, int RW>  // RW waves share a tile's rows, 4 / RW take 16 keys each
+__global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
+  using X = AtDim<D>;
+  constexpr int KG = 4 / RW, BK = 16 * KG, NB = AT_ROWS / 16 / RW;
+  __shared__ __align__(16) float lds[2 * AT_ROWS * X::P + 2 * AT_ROWS];
+  float* qt = lds;
+  float* gt = lds + AT_ROWS * X::P;
+  float* lse_t = gt + AT_ROWS * X::P;
+  float* delta_t = lse_t + AT_ROWS;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int kg = wave % KG, rw = wave / KG;
+  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const int rows = a.tq * a.rep;
+  const int j0 = blockIdx.x * BK, key = j0 + kg * 16 + i;
+  const long k_at = b * a.k_b + kvh * a.k_h + static_cast<long>(min(key, a.tk - 1)) * a.k_t;
+  float4 k[X::S], v4[X::S];
+  at_own<D>(static_cast<const float*>(a.k) + k_at, k, g);
+  at_own<D>(static_cast<const float*>(a.v) + k_at, v4, g);
+  // Queries that see key j: j .. min(T - 1, j + window - 1). Row tiles from the first key's to the last key's.
+  const int key_last = min(j0 + BK, a.tk) - 1;
+  const int q_last = a.window > 0 ? min(a.tk - 1, key_last + a.window - 1) : a.tk - 1;
+  const int u_first = j0 * a.rep / AT_ROWS, u_end = ((q_last + 1) * a.rep + AT_ROWS - 1) / AT_ROWS;
+  const int share = (u_end - u_first + gridDim.z - 1) / gridDim.z;
+  const int u0 = u_first + blockIdx.z * share, u1 = min(u_end, u0 + share);
+  const long stat_b = (static_cast<long>(b) * a.kv_heads + kvh) * a.rep;
+  AtTile<D, float> qn, gn;
+  float lse_n = 0.0f, delta_n = 0.0f;
+  auto fetch = [&](int u) {
+    auto row_of = [&](int row, long h_stride, long t_stride) {
+      const AtRow x = at_unpack(u * AT_ROWS + row, a.rep);
+      return x.head * h_stride + static_cast<long>(x.query) * t_stride;
+    };
+    const float* qb = a.q + b * a.q_b + static_cast<long>(kvh) * a.rep * a.q_h;
+    const float* gb = a.gy + b * a.o_b + static_cast<long>(kvh) * a.rep * a.o_h;
+    qn.fetch([&](int row) { return u * AT_ROWS + row < rows ? qb + row_of(row, a.q_h, a.q_t) : nullptr; });
+    gn.fetch([&](int row) { return u * AT_ROWS + row < rows ? gb + row_of(row, a.o_h, a.o_t) : nullptr; });
+    if (threadIdx.x < AT_ROWS && u * AT_ROWS + static_cast<int>(threadIdx.x) < rows) {
+      const AtRow x = at_unpack(u * AT_ROWS + threadIdx.x, a.rep);
+      const long at = (stat_b + x.head) * a.tq + x.query;
+      lse_n = a.lse[at] * AT_LOG2E;
+      delta_n = a.delta[at];
+    }
+  };
+  const AtGrad grad{a.scale, a.scale * AT_LOG2E};
+  floatx4_a dk[X::S], dv[X::S];
+#pragma unroll
+  for (int m = 0; m < X::S; ++m) dk[m] = dv[m] = at_zero();
+  bool bad = false;
+  if (u0 < u1) fetch(u0);
+  for (int u = u0; u < u1; ++u) {
+    __syncthreads();
+    qn.store(qt);
+    gn.store(gt);
+    if (threadIdx.x < AT_ROWS) {
+      lse_t[threadIdx.x] = lse_n;
+      delta_t[threadIdx.x] = delta_n;
+    }
+    __syncthreads();
+    if (u + 1 < u1) fetch(u + 1);
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const int row = (rw * NB + n) * 16;
+      const floatx4_a s = at_dot<D>(qt + row * X::P, k, i, g);
+      const floatx4_a dp = at_dot<D>(gt + row * X::P, v4, i, g);
+      const float4 l4 = *reinterpret_cast<const float4*>(lse_t + row + 4 * g);
+      const float4 d4 = *reinterpret_cast<const float4*>(delta_t + row + 4 * g);
+      const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
+      floatx4_a p, ds;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int packed = u * AT_ROWS + row + 4 * g + v, query = at_unpack(packed, a.rep).query;
+        const bool seen = packed < rows && key < a.tk && key <= query && (a.window == 0 || query < key + a.window);
+        float pv, dsv;
+        grad(seen, s[v], dp[v], lv[v], dl[v], &pv, &dsv, &bad);
+        p[v] = pv;
+        ds[v] = dsv;
+      }
+      at_accumulate<D>(gt + row * X::P, p, dv, i, g);
+      at_accumulate<D>(qt + row * X::P, ds, dk, i, g);
+    }
+  }
+  const bool split = gridDim.z > 1;
+  const long plane = static_cast<long>(a.tk) * D;  // parts: [z][b, kv head][tk][D], dK's then dV's
+  const long part_at = ((static_cast<long>(blockIdx.z) * gridDim.y + blockIdx.y) * a.tk + min(key, a.tk - 1)) * D;
+  float* ok = split ? a.parts + part_at : a.gk + k_at;
+  float* ov = split ? a.parts + static_cast<long>(gridDim.z) * gridDim.y * plane + part_at : a.gv + k_at;
+  if constexpr (RW == 1) {
+    if (key < a.tk) {
+      bad |= at_store<D, 4>(ok, dk, 1.0f, g, 0);
+      bad |= at_store<D, 4>(ov, dv, 1.0f, g, 0);
+    }
+  } else {
+    auto meet = [&](floatx4_a (&x)[X::S]) {
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < X::S; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) lds[((rw * X::S + m) * 4 + v) * 64 + lane] = x[m][v];
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < X::S; ++m) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) sum += lds[((w * X::S + m) * 4 + rw) * 64 + lane];
+        x[m] = floatx4_a{sum, sum, sum, sum};
+      }
+    };
+    meet(dk);
+    meet(dv);
+    if (key < a.tk) {
+      bad |= at_store<D, 1>(ok, dk, 1.0f, g, rw);
+      bad |= at_store<D, 1>(ov, dv, 1.0f, g, rw);
+    }
+  }
+  if (bad) dev_raise_fault(a.fault, a.tag);
+}
+
+// Adds up the parts of a split key / value pass, lowest rows first. blockIdx.y: 0 dK, 1 dV.
+__global__ __launch_bounds__(AT_THREADS) void sdpa32_parts_kernel(Sdpa32Args a, int parts, int dim, long total) {
+  const long n = static_cast<long>(blockIdx.x) * AT_THREADS + threadIdx.x;  // a 16-byte piece
+  if (n * 4 >= total) return;
+  const float* src = a.parts + static_cast<long>(blockIdx.y) * parts * total + n * 4;
+  float4 t = *reinterpret_cast<const float4*>(src);
+  for (int z = 1; z < parts; ++z) {
+    const float4 u = *reinterpret_cast<const float4*>(src + z * total);
+    t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w;
+  }
+  const long row = n * 4 / dim, plane = row / a.tk;
+  const long b = plane / a.kv_heads, kvh = plane - b * a.kv_heads;
+  float* dst = (blockIdx.y ? a.gv : a.gk) + b * a.k_b + kvh * a.k_h + (row - plane * a.tk) * a.k_t + (n * 4 - row * dim);
+  *reinterpret_cast<float4*>(dst) = t;
+  if (!(dev_finite(t.x) && dev_finite(t.y) && dev_finite(t.z) && dev_finite(t.w))) dev_raise_fault(a.fault, a.tag);
+}
+
+// Rows (keys) per workgroup: 64, or 16 with the waves splitting the other side where 64 would leave compute units
+// without a workgroup (8 x 4 heads x 256: forward 17.5 -> 12.9 us, backward 46 -> 34; 4 heads x 2048: 114 -> 69, 241 -> 190).
+bool at_narrow(omx_ctx* ctx, long planes, long rows) { return planes * ((rows + 63) / 64) < ctx->cu_count; }
+
+template <int D>
+int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) {
+  const long rows = static_cast<long>(a.tq) * a.rep;
+  const bool narrow = at_narrow(ctx, planes, rows);
+  const long bq = narrow ? 16 : 64;
+  dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
+  if (narrow) {
+    if (bf16_cache) hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 4, unsigned short>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+    else hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 4, float>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+  } else {
+    if (bf16_cache) hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 1, unsigned short>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+    else hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 1, float>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+  }
+  OMX_LAUNCH_CHECK(ctx, "sdpa32_fwd_kernel");
+  return OMX_OK;
+}
+
+template <int D>
+int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
+  const long rows = static_cast<long>(a.tq) * a.rep;
+  {
+    const bool narrow = at_narrow(ctx, planes, rows);
+    const long bq = narrow ? 16 : 64;
+    dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
+    if (narrow) hipLaunchKernelGGL((sdpa32_dq_kernel<D, 4>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+    else hipLaunchKernelGGL((sdpa32_dq_kernel<D, 1>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+    OMX_LAUNCH_CHECK(ctx, "sdpa32_dq_kernel");
+  }
+  const bool narrow = at_narrow(ctx, planes, a.tk);
+  const long bk = narrow ? 16 : 64, blocks = (a.tk + bk - 1) / bk;
+  // Split the rows until there are two workgroups per compute unit, as long as a share keeps two tiles (a part
+  // costs its write, its read and a launch).
+  const long seen = a.window > 0 ? std::min<long>(a.tk, a.window + bk) : a.tk;
+  const long tiles = std::max<long>(1, seen * a.rep / AT_ROWS);
+  long parts = std::max<long>(1, std::min<long>(2l * ctx->cu_count / (planes * blocks), tiles / 2));
+  const long total = static_cast<long>(planes) * a.tk * D;
+  while (parts > 1 && parts * total * 8 > (256l << 20)) --parts;
+  if (parts > 1) {
+    void* ws = nullptr;
+    int32_t rc = omx_workspace(ctx, static_cast<uint64_t>(parts) * total * 8, &ws, 1);
+    if (rc != OMX_OK) return rc;
+    a.parts = static_cast<float*>(ws);
+  }
+  dim3 grid(static_cast<unsigned>(blocks), planes, static_cast<unsigned>(parts));
+  if (narrow) hipLaunchKernelGGL((sdpa32_dkv_kernel<D, 4>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+  else hipLaunchKernelGGL((sdpa32_dkv_kernel<D, 1>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+  OMX_LAUNCH_CHECK(ctx, "sdpa32_dkv_kernel");
+  if (parts > 1) {
+    hipLaunchKernelGGL(sdpa32_parts_kernel, dim3(static_cast<unsigned>((total / 4 + AT_THREADS - 1) / AT_THREADS), 2), dim3(AT_THREADS), 0,
+                       ctx->stream, a, static_cast<int>(parts), D, total);
+    OMX_LAUNCH_CHECK(ctx, "sdpa32_parts_kernel");
+  }
+  return OMX_OK;
+}
+
+}  // namespace
+
+bool omx_sdpa32_supports(uint64_t dim, uint64_t planes, std::initializer_list<const void*> ptrs, std::initializer_list<long> strides) {
+  if ((dim != 16 && dim != 32 && dim != 64 && dim != 128) || planes > 65535) return false;
+  for (const void* p : ptrs)
+    if (reinterpret_cast<uintptr_t>(p) & 15u) return false;
+  for (long s : strides)
+    if (s % 4 != 0) return false;
+  return true;
+}
+
+int32_t omx_sdpa32_forward(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache) {
+  const int planes = batch * a.kv_heads;
+  if (dim == 16) return forward<16>(ctx, a, planes, bf16_cache);
+  if (dim == 32) return forward<32>(ctx, a, planes, bf16_cache);
+  if (dim == 64) return forward<64>(ctx, a, planes, bf16_cache);
+  return forward<128>(ctx, a, planes, bf16_cache);
+}
+
+int32_t omx_sdpa32_backward(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim) {
+  const int planes = batch * a.kv_heads;
+  if (dim == 16) return backward<16>(ctx, a, planes);
+  if (dim == 32) return backward<32>(ctx, a, planes);
+  if (dim == 64) return backward<64>(ctx, a, planes);
+  return backward<128>(ctx, a, planes);
+}

@@ -184,3 +184,22 @@ def test_decode_rows_under_every_block_shape(be, b, tq, h, hkv, d, kv_len):
     want = orc.cached_attention_forward(q, k, v, kv_len)
     got = be.download(be.cached_attention_forward(be.upload(q), be.upload(k), be.upload(v), kv_len))
     assert np.abs(got - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))
+
+
+@pytest.mark.parametrize("b,tq,h,hkv,d,capacity,kv_len,window", [
+    (1, 16, 1, 1, 16, 16, 16, None), (2, 17, 4, 2, 32, 90, 81, None), (3, 5, 8, 2, 64, 70, 69, 13), (2, 64, 6, 6, 64, 300, 700, 200),
+    (1, 200, 4, 1, 128, 333, 1000, 100), (5, 96, 16, 16, 64, 128, 128, None), (2, 33, 3, 3, 64, 257, 257, 1)])
+@pytest.mark.parametrize("bf16_cache", [False, True])
+def test_prompt_chunks_on_the_matrix_units(be, b, tq, h, hkv, d, capacity, kv_len, window, bf16_cache):
+    """Chunks of 16 rows per KV head and more: rings that have wrapped, windows that start inside a tile, grouped
+    heads, both block shapes, rows that end inside a block."""
+    r = np.random.default_rng(tq * 7 + d)
+    q = r.standard_normal((b, tq, h, d)).astype(np.float32)
+    seq = [r.standard_normal((b, kv_len, hkv, d)).astype(np.float32) for _ in range(2)]
+    if bf16_cache:
+        seq = [orc.round_bf16(x) for x in seq]
+    k, v = (ring(x, capacity, kv_len, 0.0) for x in seq)
+    want = orc.cached_attention_forward(q, k, v, kv_len, window or 0)
+    dk, dv = (be.upload(x, BF16) if bf16_cache else be.upload(x) for x in (k, v))
+    got = be.download(be.cached_attention_forward(be.upload(q), dk, dv, kv_len, window))
+    assert np.abs(got - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))

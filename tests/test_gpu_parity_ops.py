@@ -857,3 +857,21 @@ def test_argmax_of_rows_at_every_alignment(be, cols):
     x[1, :] = -7.0
     x[2, [cols // 3, cols - 1]] = 9.0
     assert np.array_equal(be.download(be.argmax_rows(be.upload(x))), np.argmax(x, axis=1).astype(np.uint32))
+
+
+@pytest.mark.parametrize("b,h,hkv,t,d,window", [(1, 1, 1, 1, 64, None), (2, 3, 3, 65, 16, None), (1, 8, 2, 130, 64, 17), (3, 6, 1, 200, 32, None),
+                                                (1, 2, 2, 333, 128, 64), (20, 16, 8, 64, 64, None), (1, 4, 1, 700, 64, None)])
+def test_f32_attention_on_the_matrix_units(be, b, h, hkv, t, d, window):
+    """Both block shapes (64 rows, or 16 with the waves splitting the keys), grouped rows packed across tiles, a window
+    that starts inside a tile, key / value parts added up by a second launch."""
+    r = orc.SplitMix64(1200 + t)
+    q, gy = (r.vec(b * h * t * d, 1.0).reshape(b, h, t, d) for _ in range(2))
+    k, v = (r.vec(b * hkv * t * d, 1.0).reshape(b, hkv, t, d) for _ in range(2))
+    want, want_lse = orc.causal_sdpa_forward(q, k, v, window or 0)
+    grads = orc.causal_sdpa_backward(q, k, v, want, want_lse, gy, window or 0)
+    dq, dk, dv, dg = (be.upload(x) for x in (q, k, v, gy))
+    out, lse = be.causal_sdpa_forward(dq, dk, dv, window)
+    assert np.abs(be.download(out) - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))
+    assert np.abs(be.download(lse) - want_lse).max() <= 1e-5 * max(1.0, float(np.abs(want_lse).max()))
+    for got, ref in zip(be.causal_sdpa_backward(dq, dk, dv, out, lse, dg, window), grads):
+        assert np.abs(be.download(got) - ref).max() <= 1e-5 * max(1.0, float(np.abs(ref).max()))
