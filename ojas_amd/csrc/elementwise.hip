@@ -6,6 +6,8 @@
 // (backend.rs:1115-1220,1473-1510; CPU reference ojas-cpu/src/accum.rs:31-106,
 // pointwise.rs:1052, layout.rs:82-118, ojas-core/src/erf_exact.rs:29-110,
 // gelu_tanh.rs:27-68).
+#include <algorithm>
+
 #include "omx_common.h"
 
 namespace {
@@ -13,17 +15,23 @@ namespace {
 constexpr int EW_THREADS = 256;
 constexpr int EW_PER_THREAD = 8;
 
+// Eight elements per thread, or fewer where that would make under 1024 blocks: a thread's elements follow
+// one another, and a small tensor is bound by that chain (a permute of 2 MB: 7.0 us on 64 blocks, 3.6 on 512).
 inline dim3 ew_grid(uint64_t n) {
-  uint64_t per_block = static_cast<uint64_t>(EW_THREADS) * EW_PER_THREAD;
+  const uint64_t per_block = static_cast<uint64_t>(EW_THREADS) * EW_PER_THREAD;
   uint64_t blocks = (n + per_block - 1) / per_block;
+  if (blocks < 1024) blocks = std::min<uint64_t>(1024, (n + EW_THREADS - 1) / EW_THREADS);
   return dim3(static_cast<unsigned>(blocks > 0 ? blocks : 1));
 }
 
-// Block b owns elements [b*2048, (b+1)*2048); thread t touches t, t+256, ...
-// so a wave's accesses are contiguous.
-#define EW_LOOP(i, n)                                                                      \
-  for (size_t i = static_cast<size_t>(blockIdx.x) * (EW_THREADS * EW_PER_THREAD) + threadIdx.x, \
-              end_ = min(static_cast<size_t>(n), (static_cast<size_t>(blockIdx.x) + 1) * (EW_THREADS * EW_PER_THREAD)); \
+// A block owns an equal run of elements (a multiple of 256); thread t touches t, t+256, ... of it, so a wave's
+// accesses are contiguous.
+__device__ __forceinline__ size_t ew_run(size_t n) {
+  return ((n + gridDim.x - 1) / gridDim.x + EW_THREADS - 1) / EW_THREADS * EW_THREADS;
+}
+#define EW_LOOP(i, n)                                                                                     \
+  for (size_t run_ = ew_run(n), i = static_cast<size_t>(blockIdx.x) * run_ + threadIdx.x,                 \
+              end_ = min(static_cast<size_t>(n), (static_cast<size_t>(blockIdx.x) + 1) * run_);           \
        i < end_; i += EW_THREADS)
 
 template <typename S, typename D>
