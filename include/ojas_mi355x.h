@@ -281,6 +281,21 @@ int32_t omx_causal_attention_backward_saved(omx_ctx* ctx, const void* q, uint64_
                                             uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
                                             uint64_t window);
 
+/* causal_attention of the f32 tier, time-major as above: every tensor f32, head_dim 16 / 32 / 64 / 128 (other
+ * shapes return Unsupported and the caller composes omx_permute_0213 with omx_causal_sdpa_*), pitches
+ * multiples of 4. lse is [batch, heads, time]. For a step driver that keeps q, k and v as column blocks of one
+ * projection output. */
+int32_t omx_causal_attention_f32_forward(omx_ctx* ctx, const void* q, uint64_t q_pitch, const void* k,
+                                         const void* v, uint64_t kv_pitch, void* out, uint64_t out_pitch,
+                                         void* lse, uint64_t batch, uint64_t time, uint64_t heads,
+                                         uint64_t kv_heads, uint64_t head_dim, uint64_t window);
+int32_t omx_causal_attention_f32_backward(omx_ctx* ctx, const void* q, uint64_t q_pitch, const void* k,
+                                          const void* v, uint64_t kv_pitch, const void* out,
+                                          const void* gy, uint64_t out_pitch, const void* lse, void* gq,
+                                          void* gk, void* gv, uint64_t batch, uint64_t time,
+                                          uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
+                                          uint64_t window);
+
 /* ---- BackendModule::rms_norm_forward / _backward (backend.rs:1658-1672) ---- */
 int32_t omx_rms_norm_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* w_f32,
                              void* y, int32_t y_dtype, uint64_t rows, uint64_t dim, float eps);

@@ -98,6 +98,8 @@ extern "C" {
     pub fn omx_causal_attention_backward(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, out: *const c_void, gy: *const c_void, out_pitch: u64, lse: *const c_void, operand_dtype: i32, gq: *mut c_void, gk: *mut c_void, gv: *mut c_void, grad_dtype: i32, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
     pub fn omx_causal_attention_forward_saving(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, operand_dtype: i32, out: *mut c_void, out_residual: *mut c_void, out_pitch: u64, out_dtype: i32, lse: *mut c_void, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
     pub fn omx_causal_attention_backward_saved(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, out: *const c_void, out_residual: *const c_void, gy: *const c_void, out_pitch: u64, lse: *const c_void, operand_dtype: i32, gq: *mut c_void, gk: *mut c_void, gv: *mut c_void, grad_dtype: i32, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
+    pub fn omx_causal_attention_f32_forward(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, out: *mut c_void, out_pitch: u64, lse: *mut c_void, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
+    pub fn omx_causal_attention_f32_backward(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, out: *const c_void, gy: *const c_void, out_pitch: u64, lse: *const c_void, gq: *mut c_void, gk: *mut c_void, gv: *mut c_void, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
     pub fn omx_rms_norm_forward(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, w_f32: *const c_void, y: *mut c_void, y_dtype: i32, rows: u64, dim: u64, eps: f32) -> i32;
     pub fn omx_rms_norm_backward(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, w_f32: *const c_void, gy: *const c_void, gy_dtype: i32, gx: *mut c_void, gx_dtype: i32, gw_f32: *mut c_void, rows: u64, dim: u64, eps: f32) -> i32;
     pub fn omx_residual_add_rms_norm_forward(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, y: *const c_void, y_dtype: i32, w_f32: *const c_void, sum_f32: *mut c_void, normed: *mut c_void, normed_dtype: i32, rows: u64, dim: u64, eps: f32) -> i32;

@@ -633,4 +633,64 @@ int32_t omx_causal_attention_backward_saved(omx_ctx* ctx, const void* q, uint64_
                             gq, gk, gv, grad_dtype, batch, time, heads, kv_heads, head_dim, window);
 }
 
+static int32_t attention_f32(omx_ctx* ctx, const char* op, uint32_t fault, const void* q, uint64_t q_pitch, const void* k,
+                             const void* v, uint64_t kv_pitch, uint64_t out_pitch, uint64_t batch, uint64_t time, uint64_t heads,
+                             uint64_t kv_heads, uint64_t head_dim, uint64_t window, std::initializer_list<const void*> ptrs, Sdpa32Args* a) {
+  for (const void* p : ptrs)
+    if (!p) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  SdpaShape s;
+  int32_t rc = check_shape(ctx, op, batch, heads, kv_heads, time, head_dim, window, &s);
+  if (rc != OMX_OK) return rc;
+  if (q_pitch < heads * head_dim || out_pitch < heads * head_dim || kv_pitch < kv_heads * head_dim)
+    return omx_fail(ctx, OMX_SHAPE, "%s: row pitch below heads * head_dim", op);
+  const long qp = static_cast<long>(q_pitch), kp = static_cast<long>(kv_pitch), op_ = static_cast<long>(out_pitch);
+  if (!omx_sdpa32_supports(head_dim, batch * kv_heads, ptrs, {qp, kp, op_}))
+    return omx_fail(ctx, OMX_UNSUPPORTED, "%s: head_dim %llu (16, 32, 64 or 128), 16-byte aligned tensors and pitches", op,
+                    (unsigned long long)head_dim);
+  *a = sdpa32_args(ctx, q, k, v, s, omx_tag(ctx, fault));
+  a->q_h = a->k_h = a->o_h = s.dim;
+  a->q_t = qp;
+  a->k_t = kp;
+  a->o_t = op_;
+  a->q_b = qp * s.time;
+  a->k_b = kp * s.time;
+  a->o_b = op_ * s.time;
+  return OMX_OK;
+}
+
+int32_t omx_causal_attention_f32_forward(omx_ctx* ctx, const void* q, uint64_t q_pitch, const void* k, const void* v, uint64_t kv_pitch,
+                                         void* out, uint64_t out_pitch, void* lse, uint64_t batch, uint64_t time, uint64_t heads,
+                                         uint64_t kv_heads, uint64_t head_dim, uint64_t window) {
+  OMX_REQUIRE_CTX(ctx);
+  Sdpa32Args a;
+  int32_t rc = attention_f32(ctx, "causal_attention_f32_forward", F_SDPA_FORWARD, q, q_pitch, k, v, kv_pitch, out_pitch, batch, time, heads,
+                             kv_heads, head_dim, window, {q, k, v, out, lse}, &a);
+  if (rc != OMX_OK) return rc;
+  a.out = static_cast<float*>(out);
+  a.lse = static_cast<float*>(lse);
+  return omx_sdpa32_forward(ctx, a, static_cast<int>(batch), static_cast<int>(head_dim), false);
+}
+
+int32_t omx_causal_attention_f32_backward(omx_ctx* ctx, const void* q, uint64_t q_pitch, const void* k, const void* v, uint64_t kv_pitch,
+                                          const void* out, const void* gy, uint64_t out_pitch, const void* lse, void* gq, void* gk, void* gv,
+                                          uint64_t batch, uint64_t time, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
+                                          uint64_t window) {
+  OMX_REQUIRE_CTX(ctx);
+  Sdpa32Args a;
+  int32_t rc = attention_f32(ctx, "causal_attention_f32_backward", F_SDPA_BACKWARD, q, q_pitch, k, v, kv_pitch, out_pitch, batch, time,
+                             heads, kv_heads, head_dim, window, {q, k, v, out, gy, lse, gq, gk, gv}, &a);
+  if (rc != OMX_OK) return rc;
+  void* ws = nullptr;
+  rc = omx_workspace(ctx, batch * heads * time * sizeof(float), &ws);
+  if (rc != OMX_OK) return rc;
+  a.out = const_cast<float*>(static_cast<const float*>(out));  // read only
+  a.lse = const_cast<float*>(static_cast<const float*>(lse));
+  a.gy = static_cast<const float*>(gy);
+  a.gq = static_cast<float*>(gq);
+  a.gk = static_cast<float*>(gk);
+  a.gv = static_cast<float*>(gv);
+  a.delta = static_cast<float*>(ws);
+  return omx_sdpa32_backward(ctx, a, static_cast<int>(batch), static_cast<int>(head_dim));
+}
+
 }  // extern "C"

@@ -69,9 +69,9 @@ struct ogpt {
   void *gu = nullptr, *gg = nullptr;         // [N,mlp] AD
   void *gq = nullptr, *gk = nullptr, *gv = nullptr, *ga = nullptr;  // [N,d] AD
   void* gy16 = nullptr;                      // AD copy of a residual-stream gradient
-  // bf16 tier with head_dim 64: q, k and v are column blocks of one [N, 3d] projection output
-  // (the three weights are adjacent in the arena, so they are one [3d, d] matrix), attention
-  // runs time-major on those blocks, and their gradients are the blocks of `gqkv`.
+  // Where the time-major attention takes the head dim: q, k and v are column blocks of one [N, 3d]
+  // projection output (the three weights are adjacent in the arena, so they are one [3d, d] matrix),
+  // attention runs on those blocks, and their gradients are the blocks of `gqkv`.
   bool fused_qkv = false;
   void* gqkv = nullptr;                      // [N,3d] AD
   // With the fused projection, the four weight gradients of every layer wait until the backward's
@@ -154,9 +154,11 @@ int32_t forward(ogpt* t) {
     const float* next_norm = t->w32(last ? t->nf() : t->li(l + 1, 0));
     if (t->fused_qkv) {
       TRY(omx_linear_forward(ctx, A.h1, AD, t->w(t->li(l, 1)), AD, A.q, AD, N, d, 3 * d));
-      // The output's rounding residual is kept for the backward's row term, as the reference keeps
+      // bf16: the output's rounding residual is kept for the backward's row term, as the reference keeps
       // its saved output unrounded (ojas-core/src/autocast.rs:177-186).
-      TRY(omx_causal_attention_forward_saving(ctx, A.q, 3 * d, A.k, A.v, 3 * d, AD, A.ap, A.apr, d, AD, A.lse, B, T, H,
+      if (AD == OMX_F32)
+        TRY(omx_causal_attention_f32_forward(ctx, A.q, 3 * d, A.k, A.v, 3 * d, A.ap, d, A.lse, B, T, H, H, D, 0));
+      else TRY(omx_causal_attention_forward_saving(ctx, A.q, 3 * d, A.k, A.v, 3 * d, AD, A.ap, A.apr, d, AD, A.lse, B, T, H,
                                               H, D, 0));
     } else {
       TRY(omx_linear_forward(ctx, A.h1, AD, t->w(t->li(l, 1)), AD, t->t_a, AD, N, d, d));
@@ -196,17 +198,20 @@ int32_t backward(ogpt* t) {
   const uint64_t chunk_rows = N < 16384 ? N : 16384;
   TRY(omx_linear_cross_entropy_mean(ctx, t->hf, t->w(0), AD, t->targets, N, d, c.vocab, 0, 0, chunk_rows, c.vocab,
                                     t->loss, t->ghf, AD, t->g(0)));
-  TRY(omx_rms_norm_backward(ctx, t->x_final, OMX_F32, t->w32(t->nf()), t->ghf, AD, t->gres, OMX_F32, t->g(t->nf()), N, d,
-                            eps));
-  // `gy` is the residual-stream gradient as a GEMM operand: gres itself on the f32 tier, its bf16
-  // copy (written by the kernel that produced gres) on the bf16 tier.
-  const bool defer = t->deferred_dw;  // implies the bf16 tier with the fused projection
+  // `gy` is the residual-stream gradient as a GEMM operand: the gradient itself on the f32 tier, its
+  // bf16 copy (written by the kernel that produced it) on the bf16 tier. With deferred weight gradients
+  // every layer's operands are kept: the f32 tier then forms the gradients in their kept places.
+  const bool defer = t->deferred_dw;  // implies the fused projection
+  const bool keep32 = defer && AD == OMX_F32;
   // Layer l's slice of a stacked [layers][per_layer] operand buffer.
   auto slice = [&](void* all, uint64_t l, uint64_t per_layer) {
     return static_cast<void*>(static_cast<char*>(all) + l * per_layer * t->asz);
   };
+  float* gres = keep32 ? static_cast<float*>(slice(t->gyd_all, c.layers - 1, N * d)) : t->gres;
+  TRY(omx_rms_norm_backward(ctx, t->x_final, OMX_F32, t->w32(t->nf()), t->ghf, AD, gres, OMX_F32, t->g(t->nf()), N, d,
+                            eps));
   const void* gy = nullptr;
-  TRY(to_operand(t, t->gres, defer ? slice(t->gyd_all, c.layers - 1, N * d) : t->gy16, N * d, &gy));
+  TRY(to_operand(t, gres, defer ? slice(t->gyd_all, c.layers - 1, N * d) : t->gy16, N * d, &gy));
   void* copy16 = AD == OMX_BF16 ? t->gy16 : nullptr;
   for (uint32_t l = c.layers; l-- > 0;) {
     ogpt::Layer& A = t->layers[l];
@@ -214,8 +219,10 @@ int32_t backward(ogpt* t) {
     void* gqkv = defer ? slice(t->gqkv_all, l, 3 * N * d) : t->gqkv;
     // Where the two norm backwards of this layer leave the bf16 copy of the gradient they produce:
     // the operand of this layer's o projection, and of the layer below's down projection.
-    void* copy_o = defer ? slice(t->gyo_all, l, N * d) : copy16;
-    void* copy_below = defer && l > 0 ? slice(t->gyd_all, l - 1, N * d) : copy16;
+    void* copy_o = defer && !keep32 ? slice(t->gyo_all, l, N * d) : copy16;
+    void* copy_below = defer && !keep32 && l > 0 ? slice(t->gyd_all, l - 1, N * d) : copy16;
+    float* gres1 = keep32 ? static_cast<float*>(slice(t->gyo_all, l, N * d)) : t->gres1;
+    float* below = keep32 && l > 0 ? static_cast<float*>(slice(t->gyd_all, l - 1, N * d)) : t->gres;
     // Weight gradients go to the arena now, or wait for the batched products after the loop.
     auto gw = [&](uint64_t which) { return defer ? nullptr : t->g(t->li(l, which)); };
     // x_next = x1 + down(gelu(up(norm2(x1))))
@@ -224,26 +231,30 @@ int32_t backward(ogpt* t) {
       if (!defer) TRY(omx_linear_backward(ctx, A.g, nullptr, gy, AD, nullptr, AD, t->g(t->li(l, 7)), OMX_F32, N, M, d));
       TRY(omx_linear_backward_input_gelu(ctx, t->w(t->li(l, 7)), gy, AD, A.u, gu, N, M, d, c.gelu_tanh));
     } else {
-      TRY(omx_linear_backward(ctx, A.g, t->w(t->li(l, 7)), gy, AD, t->gg, AD, t->g(t->li(l, 7)), OMX_F32, N, M, d));
+      TRY(omx_linear_backward(ctx, A.g, t->w(t->li(l, 7)), gy, AD, t->gg, AD, gw(7), OMX_F32, N, M, d));
       TRY(omx_gelu_backward(ctx, A.u, t->gg, gu, AD, N * M, c.gelu_tanh));
     }
     TRY(omx_linear_backward(ctx, A.h2, t->w(t->li(l, 6)), gu, AD, t->t_a, AD, gw(6), OMX_F32, N, d, M));
     // Fan-in at x1: the residual branch arrives first, then the norm branch.
-    TRY(omx_rms_norm_backward_residual(ctx, A.x1, OMX_F32, t->w32(t->li(l, 5)), t->t_a, AD, t->gres, t->gres1, copy_o,
+    TRY(omx_rms_norm_backward_residual(ctx, A.x1, OMX_F32, t->w32(t->li(l, 5)), t->t_a, AD, gres, gres1, copy_o,
                                        t->g(t->li(l, 5)), N, d, eps));
-    gy = AD == OMX_BF16 ? static_cast<const void*>(copy_o) : static_cast<const void*>(t->gres1);
+    gy = AD == OMX_BF16 ? static_cast<const void*>(copy_o) : static_cast<const void*>(gres1);
     // x1 = x + o(attention)
     TRY(omx_linear_backward(ctx, A.ap, t->w(t->li(l, 4)), gy, AD, t->t_a, AD, gw(4), OMX_F32, N, d, d));
     if (t->fused_qkv) {
       char* gq = static_cast<char*>(gqkv);
-      TRY(omx_causal_attention_backward_saved(ctx, A.q, 3 * d, A.k, A.v, 3 * d, A.ap, A.apr, t->t_a, d, A.lse, AD, gq,
+      if (AD == OMX_F32)
+        TRY(omx_causal_attention_f32_backward(ctx, A.q, 3 * d, A.k, A.v, 3 * d, A.ap, t->t_a, d, A.lse, gq, gq + d * t->asz,
+                                              gq + 2 * d * t->asz, B, T, H, H, D, 0));
+      else TRY(omx_causal_attention_backward_saved(ctx, A.q, 3 * d, A.k, A.v, 3 * d, A.ap, A.apr, t->t_a, d, A.lse, AD, gq,
                                         gq + d * t->asz, gq + 2 * d * t->asz, AD, B, T, H, H, D, 0));
       // One product for the three projections: the input gradient is their sum, formed in the
       // product's f32 accumulators.
       TRY(omx_linear_backward(ctx, A.h1, t->w(t->li(l, 1)), gqkv, AD, t->t_b, AD, gw(1), OMX_F32, N, d, 3 * d));
-      TRY(omx_rms_norm_backward_residual(ctx, A.x, OMX_F32, t->w32(t->li(l, 0)), t->t_b, AD, t->gres1, t->gres,
+      TRY(omx_rms_norm_backward_residual(ctx, A.x, OMX_F32, t->w32(t->li(l, 0)), t->t_b, AD, gres1, below,
                                          copy_below, t->g(t->li(l, 0)), N, d, eps));
-      gy = AD == OMX_BF16 ? static_cast<const void*>(copy_below) : static_cast<const void*>(t->gres);
+      gres = below;
+      gy = AD == OMX_BF16 ? static_cast<const void*>(copy_below) : static_cast<const void*>(gres);
       continue;
     }
     TRY(omx_permute_0213(ctx, t->t_a, t->ga, AD, B, T, H, D));
@@ -257,7 +268,7 @@ int32_t backward(ogpt* t) {
     TRY(omx_permute_0213(ctx, t->gq, t->t_a, AD, B, H, T, D));
     TRY(omx_linear_backward(ctx, A.h1, t->w(t->li(l, 1)), t->t_a, AD, t->ga, AD, t->g(t->li(l, 1)), OMX_F32, N, d, d));
     TRY(omx_residual_add(ctx, t->gh, OMX_F32, t->ga, AD, t->gh, OMX_F32, N * d));
-    TRY(omx_rms_norm_backward_residual(ctx, A.x, OMX_F32, t->w32(t->li(l, 0)), t->gh, OMX_F32, t->gres1, t->gres, copy16,
+    TRY(omx_rms_norm_backward_residual(ctx, A.x, OMX_F32, t->w32(t->li(l, 0)), t->gh, OMX_F32, gres1, t->gres, copy16,
                                        t->g(t->li(l, 0)), N, d, eps));
     gy = AD == OMX_BF16 ? static_cast<const void*>(t->gy16) : static_cast<const void*>(t->gres);
   }
@@ -278,9 +289,9 @@ int32_t backward(ogpt* t) {
                                  0, layers, N * p.out, N * p.in, per_layer));
   }
   // x0 = tok[ids] + pos[positions]; the tied table adds the embedding's share to the head's.
-  TRY(omx_embedding_backward(ctx, t->positions, t->gres, OMX_F32, t->g(1), N, T, d));
+  TRY(omx_embedding_backward(ctx, t->positions, gres, OMX_F32, t->g(1), N, T, d));
   // The tied table: the gather's gradient joins the head's where it lies, row by named row.
-  TRY(omx_embedding_backward_accumulate(ctx, t->ids, t->gres, OMX_F32, t->g(0), N, c.vocab, d));
+  TRY(omx_embedding_backward_accumulate(ctx, t->ids, gres, OMX_F32, t->g(0), N, c.vocab, d));
   return OMX_OK;
 }
 
@@ -331,7 +342,8 @@ int32_t ogpt_create(omx_ctx* ctx, const ogpt_config* config, ogpt** out) {
   for (uint64_t l = 0; l < c.layers; ++l)
     for (uint64_t w : {1, 2, 3, 4, 6, 7}) place(t->li(l, w));
   // wq, wk, wv sit back to back when d*d needs no padding.
-  t->fused_qkv = c.bf16 && c.head_dim == 64 && (d * d) % kAlign == 0;
+  const bool head_dim_fits = c.head_dim == 64 || c.head_dim == 128 || (!c.bf16 && (c.head_dim == 16 || c.head_dim == 32));
+  t->fused_qkv = head_dim_fits && (d * d) % kAlign == 0;
   auto fail = [&](int32_t rc) {
     ogpt_destroy(t);
     return rc;
@@ -403,7 +415,7 @@ int32_t ogpt_create(omx_ctx* ctx, const ogpt_config* config, ogpt** out) {
       A.k = static_cast<char*>(A.q) + d * t->asz;
       A.v = static_cast<char*>(A.q) + 2 * d * t->asz;
       A.a = nullptr;
-      CREATE_TRY(alloc_act(t, N * d, &A.apr));
+      if (c.bf16) CREATE_TRY(alloc_act(t, N * d, &A.apr));
     } else {
       CREATE_TRY(alloc_act(t, N * d, &A.q));
       CREATE_TRY(alloc_act(t, N * d, &A.k));
