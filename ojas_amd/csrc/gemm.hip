@@ -407,7 +407,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a_rs, uint64_t a_cs, const void* b,
                       uint64_t b_rs, uint64_t b_cs, int32_t operand_dtype, void* c, int32_t c_dtype, uint64_t ldc,
                       uint64_t m, uint64_t k, uint64_t n, int32_t accumulate, const OmxGemmEpilogue* epi,
-                      const OmxGemmBatch* batch) {
+                      const OmxGemmBatch* batch, uint64_t a_k) {
   const char* op = omx_fault_name(fault_op);
   const uint64_t batches = batch ? batch->count : 1;
   if (batches == 0 || batches > 65535) return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: 1..65535 products per launch", op);
@@ -450,7 +450,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   g.ldc = static_cast<long>(ldc);
   g.M = static_cast<int>(m);
   g.N = static_cast<int>(n);
-  g.K = static_cast<int>(k);
+  g.K = g.k_rows = static_cast<int>(k);
+  g.a_k = a_k > k && a_k <= 0x7fffffffull ? static_cast<int>(a_k) : g.K;
   g.c_bf16 = c_dtype == OMX_BF16;
   g.accumulate = accumulate;
   g.a_vec = aligned16(a) && (lda % kv == 0);
@@ -510,7 +511,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       const long cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
       const long tiles256 = static_cast<long>((g.M + 255) / 256) * ((g.N + 255) / 256);
       const long tiles128 = static_cast<long>((g.M + 127) / 128) * ((g.N + 127) / 128);
-      const long ksteps64 = g.K / 64;
+      const long ksteps64 = (g.K + 63) / 64;
       // How full the last round of 256 x 256 tiles is, one workgroup per compute unit.
       const long all256 = tiles256 * g.batches;
       const long rounds256 = (all256 + cus - 1) / cus;
@@ -580,18 +581,23 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       ctx->gemm_in_row_split = true;
       ctx->gemm_forced_tiling = dma_variant;
       int32_t rc = omx_gemm_impl(ctx, fault_op, a, a_rs, a_cs, b, b_rs, b_cs, operand_dtype, c, c_dtype, ldc, m0, k, n,
-                                 accumulate, epi, nullptr);
+                                 accumulate, epi, nullptr, a_k);
       ctx->gemm_forced_tiling = -1;
       if (rc == OMX_OK)
         rc = omx_gemm_impl(ctx, fault_op, static_cast<const char*>(a) + m0 * a_rs * esz, a_rs, a_cs, b, b_rs, b_cs,
                            operand_dtype, static_cast<char*>(c) + m0 * ldc * csz, c_dtype, ldc, m - m0, k, n,
-                           accumulate, epi, nullptr);
+                           accumulate, epi, nullptr, a_k);
       ctx->gemm_in_row_split = false;
       return rc;
     }
   }
   int BM = 128, BN = 128;
-  if (dma_variant >= 0) omx_gemm_dma_tile(dma_variant, &BM, &BN);
+  if (dma_variant >= 0) {
+    omx_gemm_dma_tile(dma_variant, &BM, &BN);
+    // Whole K steps: pairs of 64 columns for the one-wave-per-SIMD kernel, 64 for the others.
+    const int step = dma_variant >= 9 ? 128 : 64;
+    g.K = (g.k_rows + step - 1) / step * step;
+  }
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.N + BN - 1) / BN;
   if (static_cast<long>(g.tiles_m) * g.tiles_n > 0x7fffffffl)

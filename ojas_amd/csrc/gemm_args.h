@@ -9,6 +9,8 @@ struct GemmArgs {
   void* c;
   long lda, ldb, ldc;
   int M, N, K;
+  int k_rows;  // direct-to-LDS kernels: K is rounded up to whole steps, k-major operands end after k_rows rows
+  int a_k;     // columns of a k-contiguous A's rows that may be read (zeros past K); K itself otherwise
   int c_bf16, accumulate;
   int a_vec, b_vec;  // 16-byte loads allowed (alignment of base and leading dimension)
   int c_vec;         // 4-column stores allowed (alignment of C and its row pitch)
@@ -269,8 +271,8 @@ __device__ __forceinline__ bool gemm_store_block(const GemmArgs& g, int split, c
 }
 
 // bf16 kernels with direct-to-LDS loads and a 256 x 256 (variant 9), 256 x 128 (variant 3) or
-// 128 x 128 (variant 6) workgroup tile. Needs K % 64 == 0, 16-byte aligned
-// operands, and row counts that are multiples of 8 for k-major operands.
+// 128 x 128 (variant 6) workgroup tile. Needs 16-byte aligned operands, and whole K steps in the
+// rows of k-contiguous ones.
 bool omx_gemm_dma_eligible(const GemmArgs& g, bool a_km, bool b_km);
 bool omx_gemm_w4_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain);
 void omx_gemm_dma_tile(int variant, int* bm, int* bn);

@@ -36,18 +36,24 @@ int32_t omx_gemm_dma_launch_nt(omx_ctx* ctx, const GemmArgs& g, int variant);
 int32_t omx_gemm_dma_launch_tn(omx_ctx* ctx, const GemmArgs& g, int variant);
 int32_t omx_gemm_dma_launch_tt(omx_ctx* ctx, const GemmArgs& g, int variant);
 
+// K up to whole steps of `step` columns: what a k-contiguous A's rows hold (zeros past K), a k-major operand bounds by
+// itself; a k-contiguous B has to end with a step.
+static bool whole_steps(const GemmArgs& g, bool a_km, bool b_km, int step) {
+  if (g.K % step == 0) return true;
+  const long up = (static_cast<long>(g.K) + step - 1) / step * step;
+  return b_km && (a_km || g.a_k >= up) && up <= 0x7fffffffl;
+}
+
 bool omx_gemm_dma_eligible(const GemmArgs& g, bool a_km, bool b_km) {
-  if (g.K % 64 != 0 || !g.a_vec || !g.b_vec) return false;
+  if (!whole_steps(g, a_km, b_km, 64) || !g.a_vec || !g.b_vec) return false;
   if (g.lda >= (1l << 22) || g.ldb >= (1l << 22)) return false;  // a tile's lane offsets are 32 bits of bytes
-  if (a_km && g.M % 8 != 0) return false;
-  if (b_km && g.N % 8 != 0) return false;
   return true;
 }
 
 // The one-wave-per-SIMD kernel (variants 9 and 10) also needs a k-major B with a k-major A, an even
 // number of 64-column K steps, and a store pass without an activation.
 bool omx_gemm_w4_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain) {
-  return plain && (!a_km || b_km) && g.K % 128 == 0;
+  return plain && (!a_km || b_km) && whole_steps(g, a_km, b_km, 128);
 }
 
 void omx_gemm_dma_tile(int variant, int* bm, int* bn) {

@@ -78,12 +78,10 @@ gemm_dma_kernel(GemmArgs g) {
   // Everything a K step needs is computed here, once per tile: the loads' global addresses and
   // the fragments' LDS offsets. Inside the loop the stage is a compile-time constant (the loop
   // body is unrolled over the stages), so a step is loads, LDS reads and MFMAs and little else.
-  // (scalar base + lane offsets where every wave issues the same number of loads of each operand)
-  constexpr bool EVEN_LOADS = (BM * DBK * 2 / 1024) % NW == 0 && (BN * DBK * 2 / 1024) % NW == 0;
-  std::conditional_t<EVEN_LOADS, TileLoadsOff<A_KM, BM, DBK, NW>, TileLoads<A_KM, BM, DBK, NW>> la;
-  std::conditional_t<EVEN_LOADS, TileLoadsOff<B_KM, BN, DBK, NW>, TileLoads<B_KM, BN, DBK, NW>> lb;
-  la.init(A, g.lda, m0, g.M, ks_begin * DBK, wave, lane);
-  lb.init(B, g.ldb, n0, g.N, ks_begin * DBK, wave, lane);
+  TileLoadsOff<A_KM, BM, DBK, NW> la;
+  TileLoadsOff<B_KM, BN, DBK, NW> lb;
+  la.init(A, g.lda, m0, g.M, ks_begin * DBK, g.k_rows, wave, lane);
+  lb.init(B, g.ldb, n0, g.N, ks_begin * DBK, g.k_rows, wave, lane);
   const unsigned lds0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem)));
   int a_off[TM][KK], b_off[TN][KK];
 #pragma unroll

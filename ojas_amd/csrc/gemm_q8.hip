@@ -119,7 +119,7 @@ __global__ __launch_bounds__(512, 4) void gemm_q8_kernel(Q8Args g) {
 
   const int steps = g.K / QBK;
   TileLoadsOff<false, QBM, QBK, QNW> la;  // a scalar base that advances by the step and fixed lane offsets
-  la.init(g.a, g.lda, m0, g.M, 0, wave, lane);
+  la.init(g.a, g.lda, m0, g.M, 0, g.K, wave, lane);
   const unsigned lds0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem)));
 
   // This lane's 16 codes of a step, its scale, and where their 16 bf16 go in the widened tile. The

@@ -35,8 +35,6 @@ constexpr int W4_OPERAND = W4_BM * W4_BK * 2;  // one stage of one operand
 constexpr int W4_SMEM = 4 * W4_OPERAND;
 constexpr int W4_B0 = 2 * W4_OPERAND;  // LDS byte offset of B's first stage
 
-// Loads of one operand: a wave-uniform base address (the tile's first element at the current K
-// step) and a 32-bit byte offset per lane and load, so a K step advances one scalar.
 // The chunk swizzle of a k-major tile row (kr) of ROWS columns: 16-byte chunks moved by multiples of 64 bytes so that
 // the four K rows a transposing read touches per clock fall into different banks (rows of 512 bytes all start in
 // bank 0: four shifts; rows of 384 bytes alternate between banks 0 and 32: one shift for every second pair).
@@ -45,14 +43,14 @@ __device__ __forceinline__ int w4_km_swizzle(int kr) {
   return ROWS == 256 ? (kr & 3) * 4 : ((kr >> 1) & 1) * 4;
 }
 
+// Loads of one operand (see StepBase for the base address and the end of the K rows).
 template <bool KM, int ROWS>
 struct W4Loads {
   static constexpr int N = ROWS / 32;  // ROWS / 8 loads of 1 KiB per step, four waves
   unsigned off[N];
-  const char* base;
-  long step;
+  StepBase<KM> base;
   __device__ __forceinline__ void init(const unsigned short* __restrict__ p, long ld, int row0, int rows, int k0,
-                                       int wave, int lane) {
+                                       int k_rows, int wave, int lane) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int q = wave + 4 * i;
@@ -68,20 +66,16 @@ struct W4Loads {
         const int kr = idx / CPR, slot = idx % CPR;
         const int mc = slot ^ w4_km_swizzle<ROWS>(kr);
         int gm = mc * 8;
-        gm = row0 + gm + 8 <= rows ? gm : 0;
+        gm = row0 + gm < rows ? gm : 0;
         off[i] = static_cast<unsigned>(kr) * static_cast<unsigned>(ld * 2) + gm * 2;
       }
     }
-    base = reinterpret_cast<const char*>(p) +
-           (KM ? static_cast<long>(k0) * ld + row0 : static_cast<long>(row0) * ld + k0) * 2;
-    step = (KM ? W4_BK * ld : W4_BK) * 2;
+    base.init(p, ld, row0, k0, k_rows, W4_BK);
   }
   // Load I of this wave into LDS byte `lds_wave` + LDS_IMM.
   template <int I, int LDS_IMM>
   __device__ __forceinline__ void issue(unsigned lds_wave) const {
-    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off[I]), "s"(base),
-                 "s"(lds_wave), "n"(LDS_IMM)
-                 : "memory", "scc");
+    base.template load<LDS_IMM>(off[I], lds_wave);
   }
 };
 
@@ -186,8 +180,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   const int steps = ks_end - ks_begin;
   W4Loads<A_KM, W4_BM> la;
   W4Loads<B_KM, W4_BN> lb;
-  la.init(A, g.lda, m0, g.M, ks_begin * W4_BK, wave, lane);
-  lb.init(B, g.ldb, n0, g.N, ks_begin * W4_BK, wave, lane);
+  la.init(A, g.lda, m0, g.M, ks_begin * W4_BK, g.k_rows, wave, lane);
+  lb.init(B, g.ldb, n0, g.N, ks_begin * W4_BK, g.k_rows, wave, lane);
   const unsigned lds_wave =
       __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem))) + wave * 1024;
   // Waits until at most YES (if `which`) or NO of this wave's loads, the most recently issued, are in flight.
@@ -256,13 +250,13 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
     // Both stages' loads, part 0 of step 0 published, its fragments read.
     static_for<0, NP0>([&](auto n_index) { issue_p0(S0, n_index); });
     static_for<0, 4>([&](auto n_index) { issue_p1(S0, n_index); });
-    la.base += la.step;
-    lb.base += lb.step;
+    la.base.advance();
+    lb.base.advance();
     if (steps > 1) {
       static_for<0, NP0>([&](auto n_index) { issue_p0(S1, n_index); });
       static_for<0, 4>([&](auto n_index) { issue_p1(S1, n_index); });
-      la.base += la.step;
-      lb.base += lb.step;
+      la.base.advance();
+      lb.base.advance();
     }
     clear_acc();
     wait_loads(steps > 1, std::integral_constant<int, 4 + NSTEP>{}, C4{});
@@ -301,7 +295,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
           __builtin_amdgcn_sched_barrier(0);
         }
       });
-      if (loads) lb.base += lb.step;
+      if (loads) lb.base.advance();
       // B1. In flight behind part 0 of the next step: its part 1 and part 0 of the one after.
       publish(loads, C4P0{}, C4{});
       // Half 1.
@@ -316,7 +310,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
           read_p0(THERE, std::integral_constant<int, n / SL - 1>{}, std::integral_constant<int, n % SL>{});
         __builtin_amdgcn_sched_barrier(0);
       });
-      if (loads) la.base += la.step;
+      if (loads) la.base.advance();
       static_for<0, TN + 2>([&](auto n_index) { read_p0(THERE, std::integral_constant<int, 3>{}, n_index); });
       __builtin_amdgcn_sched_barrier(0);
     };
@@ -360,13 +354,13 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
 
     static_for<0, NPART>([&](auto n_index) { issue_part(S0, H0, n_index); });
     static_for<0, NPART>([&](auto n_index) { issue_part(S0, H1, n_index); });
-    la.base += la.step;
-    lb.base += lb.step;
+    la.base.advance();
+    lb.base.advance();
     if (steps > 1) {
       static_for<0, NPART>([&](auto n_index) { issue_part(S1, H0, n_index); });
       static_for<0, NPART>([&](auto n_index) { issue_part(S1, H1, n_index); });
-      la.base += la.step;
-      lb.base += lb.step;
+      la.base.advance();
+      lb.base.advance();
     }
     clear_acc();
     wait_loads(steps > 1, C3P{}, C1P{});
@@ -411,8 +405,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
         __builtin_amdgcn_sched_barrier(0);
       });
       if (loads) {
-        la.base += la.step;
-        lb.base += lb.step;
+        la.base.advance();
+        lb.base.advance();
       }
       __builtin_amdgcn_sched_barrier(0);
     };

@@ -126,7 +126,8 @@ __global__ __launch_bounds__(CE_THREADS) void ce_tile_stats_kernel(const T* __re
   const unsigned int tcol = target - col0;  // wraps to a huge value when the target is left of this tile
   float mx = -INFINITY, sum = 0.0f;
   bool bad = false;
-  for (unsigned int c = threadIdx.x * VEC; c < ncols; c += CE_THREADS * VEC) {
+  const unsigned int whole = ncols - ncols % VEC;  // whole packs; the columns past them go one per thread
+  for (unsigned int c = threadIdx.x * VEC; c < whole; c += CE_THREADS * VEC) {
     float v[VEC];
     ce_load<T, VEC>(r, c, v);
     float top = v[0];
@@ -142,6 +143,16 @@ __global__ __launch_bounds__(CE_THREADS) void ce_tile_stats_kernel(const T* __re
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
       if (c + j != tcol) sum += ce_exp<T>(v[j] - mx);
+  }
+  if (VEC > 1 && threadIdx.x < ncols - whole) {
+    const unsigned int c = whole + threadIdx.x;
+    const float v = dev_load<T>(r, c);
+    bad |= !dev_finite(v);
+    if (v > mx) {
+      sum *= ce_exp<T>(mx - v);
+      mx = v;
+    }
+    if (c != tcol) sum += ce_exp<T>(v - mx);
   }
   const float row_max = block_max(mx, red);
   sum = block_sum(mx == -INFINITY ? 0.0f : sum * expf(mx - row_max), red);
@@ -192,11 +203,13 @@ __global__ __launch_bounds__(1024) void ce_mean_kernel(CeState st, const unsigne
   }
 }
 
-// One block per row: tile of logits -> tile of gradients (may be in place).
+// One block per row: tile of logits -> tile of gradients (may be in place), zeros in columns ncols .. zero_to - 1
+// (the padding of a row that a product reads in whole K steps).
 template <typename TL, typename TG, int VEC>
 __global__ __launch_bounds__(CE_THREADS) void ce_tile_grad_kernel(const TL* __restrict__ tile, TG* __restrict__ grad,
                                                                   size_t ld, size_t ld_grad, size_t row0,
                                                                   unsigned int col0, unsigned int ncols,
+                                                                  unsigned int zero_to,
                                                                   const unsigned int* __restrict__ targets,
                                                                   int has_ignore, unsigned int ignore, CeState st,
                                                                   const unsigned int* __restrict__ valid) {
@@ -204,11 +217,14 @@ __global__ __launch_bounds__(CE_THREADS) void ce_tile_grad_kernel(const TL* __re
   const TL* r = tile + local * ld;
   TG* g = grad + local * ld_grad;
   const unsigned int target = targets[row];
+  const unsigned int whole = ncols - ncols % VEC;
+  for (unsigned int c = ncols + threadIdx.x; c < zero_to; c += CE_THREADS) dev_store<TG>(g, c, 0.0f);
   if (has_ignore && target == ignore) {
     float zero[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) zero[j] = 0.0f;
-    for (unsigned int c = threadIdx.x * VEC; c < ncols; c += CE_THREADS * VEC) ce_store<TG, VEC>(g, c, zero);
+    for (unsigned int c = threadIdx.x * VEC; c < whole; c += CE_THREADS * VEC) ce_store<TG, VEC>(g, c, zero);
+    if (VEC > 1 && threadIdx.x < ncols - whole) dev_store<TG>(g, whole + threadIdx.x, 0.0f);
     return;
   }
   const unsigned int tcol = target - col0;
@@ -219,12 +235,16 @@ __global__ __launch_bounds__(CE_THREADS) void ce_tile_grad_kernel(const TL* __re
   const float d = collapse ? 1.0f + other : sum;
   const float target_grad = collapse ? -(other / d) / denom : (expf(p - m) / d) / denom - 1.0f / denom;
   const float scale = (1.0f / d) / denom;
-  for (unsigned int c = threadIdx.x * VEC; c < ncols; c += CE_THREADS * VEC) {
+  for (unsigned int c = threadIdx.x * VEC; c < whole; c += CE_THREADS * VEC) {
     float v[VEC], out[VEC];
     ce_load<TL, VEC>(r, c, v);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) out[j] = (c + j == tcol) ? target_grad : ce_exp<TL>(v[j] - m) * scale;
     ce_store<TG, VEC>(g, c, out);
+  }
+  if (VEC > 1 && threadIdx.x < ncols - whole) {
+    const unsigned int c = whole + threadIdx.x;
+    dev_store<TG>(g, c, c == tcol ? target_grad : ce_exp<TL>(dev_load<TL>(r, c) - m) * scale);
   }
 }
 
@@ -271,7 +291,7 @@ __device__ __forceinline__ float fused_block_sum(float v, float* red) {
 }
 template <typename T, int MAXV>
 __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __restrict__ tile, size_t ld, size_t row0,
-                                                                  unsigned int ncols,
+                                                                  unsigned int ncols, unsigned int zero_to,
                                                                   const unsigned int* __restrict__ targets,
                                                                   int has_ignore, unsigned int ignore, CeState st,
                                                                   const unsigned int* __restrict__ valid,
@@ -286,11 +306,16 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
   // Every pack of the row, all loads in flight together. Packs past the end re-read the last one
   // (unconditional loads; they are masked out below).
   uint4 q[MAXV];
-  const unsigned int last = ncols - VEC;
+  const unsigned int whole = ncols - ncols % VEC, last = whole - VEC;  // whole packs (at least one)
+  // The columns past the whole packs go one to a thread; the padding of the row becomes zeros.
+  const unsigned int mine_c = whole + threadIdx.x;
+  const bool has_tail = threadIdx.x < ncols - whole;
+  const float tail = has_tail ? dev_load<T>(r, mine_c) : 0.0f;
+  for (unsigned int c = ncols + threadIdx.x; c < zero_to; c += CE_FUSED_THREADS) dev_store<T>(r, c, 0.0f);
 #pragma unroll
   for (int k = 0; k < MAXV; ++k) {
     const unsigned int c = (threadIdx.x + k * CE_FUSED_THREADS) * VEC;
-    q[k] = *reinterpret_cast<const uint4*>(r + (c < ncols ? c : last));
+    q[k] = *reinterpret_cast<const uint4*>(r + (c < whole ? c : last));
   }
   auto unpack = [](const uint4& w, float (&v)[VEC]) {
     const unsigned int u[4] = {w.x, w.y, w.z, w.w};
@@ -318,7 +343,7 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
 #pragma unroll
     for (int k = 0; k < MAXV; ++k) {
       const unsigned int c = (threadIdx.x + k * CE_FUSED_THREADS) * VEC;
-      if (c < ncols) {
+      if (c < whole) {
         float v[VEC];
         unpack(q[k], v);
         const float top = fmaxf(ce_max3(ce_max3(ce_max3(v[0], v[1], v[2]), v[3], v[4]), v[5], v[6]), v[7]);
@@ -345,7 +370,7 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
 #pragma unroll
     for (int k = 0; k < MAXV; ++k) {
       const unsigned int c = (threadIdx.x + k * CE_FUSED_THREADS) * VEC;
-      if (c < ncols) {
+      if (c < whole) {
         float v[VEC];
         unpack(q[k], v);
         float top = v[0];
@@ -366,6 +391,15 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
       }
     }
   }
+  if (has_tail) {
+    bad |= !dev_finite(tail);
+    if (tail > mx) {
+      sum *= ce_exp<T>(mx - tail);
+      mx = tail;
+    }
+    if (mine_c != target) sum += ce_exp<T>(tail - mx);
+    else picked = tail;
+  }
   const float row_max = fused_block_max(mx, red);
   sum = fused_block_sum(mx == -INFINITY ? 0.0f : sum * expf(mx - row_max), red);
   if (__syncthreads_or(bad)) {
@@ -381,8 +415,9 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
 #pragma unroll
     for (int k = 0; k < MAXV; ++k) {
       const unsigned int c = (threadIdx.x + k * CE_FUSED_THREADS) * VEC;
-      if (c < ncols) *reinterpret_cast<uint4*>(r + c) = make_uint4(0u, 0u, 0u, 0u);
+      if (c < whole) *reinterpret_cast<uint4*>(r + c) = make_uint4(0u, 0u, 0u, 0u);
     }
+    if (has_tail) dev_store<T>(r, mine_c, 0.0f);
     return;
   }
   const float denom = static_cast<float>(*valid);
@@ -391,10 +426,11 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
   const float d = collapse ? 1.0f + other : total;
   const float target_grad = collapse ? -(other / d) / denom : (expf(p - m) / d) / denom - 1.0f / denom;
   const float scale = (1.0f / d) / denom;
+  if (has_tail) dev_store<T>(r, mine_c, mine_c == target ? target_grad : ce_exp<T>(tail - m) * scale);
 #pragma unroll
   for (int k = 0; k < MAXV; ++k) {
     const unsigned int c = (threadIdx.x + k * CE_FUSED_THREADS) * VEC;
-    if (c < ncols) {
+    if (c < whole) {
       float v[VEC], out[VEC];
       unpack(q[k], v);
       if constexpr (sizeof(T) == 2) {
@@ -425,15 +461,15 @@ constexpr int CE_FUSED_PACKS = 8;  // per thread: rows of up to 65536 bf16 or 32
 
 // Whether rows of `ld` elements starting at `base` (+ col offset) allow 16-byte accesses of T.
 template <typename T>
-bool ce_vector_ok(const void* base, size_t ld, unsigned int ncols) {
-  return (reinterpret_cast<uintptr_t>(base) & 15u) == 0 && (ld * sizeof(T)) % 16 == 0 && ncols % ce_vec<T>() == 0;
+bool ce_vector_ok(const void* base, size_t ld) {
+  return (reinterpret_cast<uintptr_t>(base) & 15u) == 0 && (ld * sizeof(T)) % 16 == 0;
 }
 
 template <typename T>
 void launch_stats(omx_ctx* ctx, const void* tile, size_t ld, size_t row0, size_t nrows, unsigned int col0,
                   unsigned int ncols, const unsigned int* targets, CeState st, int first, unsigned long long tag) {
   dim3 grid(static_cast<unsigned>(nrows)), block(CE_THREADS);
-  if (ce_vector_ok<T>(tile, ld, ncols))
+  if (ce_vector_ok<T>(tile, ld))
     hipLaunchKernelGGL((ce_tile_stats_kernel<T, ce_vec<T>()>), grid, block, 0, ctx->stream,
                        static_cast<const T*>(tile), ld, row0, col0, ncols, targets, st, first, ctx->fault, tag);
   else
@@ -442,20 +478,20 @@ void launch_stats(omx_ctx* ctx, const void* tile, size_t ld, size_t row0, size_t
 }
 template <typename TL, typename TG>
 void launch_grad(omx_ctx* ctx, const void* tile, void* grad, size_t ld, size_t ld_grad, size_t row0, size_t nrows,
-                 unsigned int col0, unsigned int ncols, const unsigned int* targets, int has_ignore,
+                 unsigned int col0, unsigned int ncols, unsigned int zero_to, const unsigned int* targets, int has_ignore,
                  unsigned int ignore, CeState st, const unsigned int* valid) {
   dim3 grid(static_cast<unsigned>(nrows)), block(CE_THREADS);
   // 16-byte packs on both sides need logits and gradients of one element size.
   if constexpr (sizeof(TL) == sizeof(TG)) {
-    if (ce_vector_ok<TL>(tile, ld, ncols) && ce_vector_ok<TG>(grad, ld_grad, ncols)) {
+    if (ce_vector_ok<TL>(tile, ld) && ce_vector_ok<TG>(grad, ld_grad)) {
       hipLaunchKernelGGL((ce_tile_grad_kernel<TL, TG, ce_vec<TL>()>), grid, block, 0, ctx->stream,
-                         static_cast<const TL*>(tile), static_cast<TG*>(grad), ld, ld_grad, row0, col0, ncols, targets,
+                         static_cast<const TL*>(tile), static_cast<TG*>(grad), ld, ld_grad, row0, col0, ncols, zero_to, targets,
                          has_ignore, ignore, st, valid);
       return;
     }
   }
   hipLaunchKernelGGL((ce_tile_grad_kernel<TL, TG, 1>), grid, block, 0, ctx->stream, static_cast<const TL*>(tile),
-                     static_cast<TG*>(grad), ld, ld_grad, row0, col0, ncols, targets, has_ignore, ignore, st, valid);
+                     static_cast<TG*>(grad), ld, ld_grad, row0, col0, ncols, zero_to, targets, has_ignore, ignore, st, valid);
 }
 
 // State + valid counter carved out of a workspace block.
@@ -588,16 +624,16 @@ int32_t omx_cross_entropy_mean_backward(omx_ctx* ctx, const void* logits, int32_
                      s.valid, loss_scratch, ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "ce_mean_kernel");
   if (logits_dtype == OMX_F32 && grad_dtype == OMX_F32)
-    launch_grad<float, float>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, tg, has_ignore, ignore_index, s.st,
+    launch_grad<float, float>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, vocab, tg, has_ignore, ignore_index, s.st,
                               s.valid);
   else if (logits_dtype == OMX_F32)
-    launch_grad<float, unsigned short>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, tg, has_ignore,
+    launch_grad<float, unsigned short>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, vocab, tg, has_ignore,
                                        ignore_index, s.st, s.valid);
   else if (grad_dtype == OMX_F32)
-    launch_grad<unsigned short, float>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, tg, has_ignore,
+    launch_grad<unsigned short, float>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, vocab, tg, has_ignore,
                                        ignore_index, s.st, s.valid);
   else
-    launch_grad<unsigned short, unsigned short>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, tg, has_ignore,
+    launch_grad<unsigned short, unsigned short>(ctx, logits, grad, vocab, vocab, 0, rows, 0, vocab, vocab, tg, has_ignore,
                                                 ignore_index, s.st, s.valid);
   OMX_LAUNCH_CHECK(ctx, "ce_tile_grad_kernel");
   return OMX_OK;
@@ -623,8 +659,13 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
   const bool one_tile = C >= vocab;
   const bool want_grads = gx || gw;
   const size_t esz = omx_dtype_size(operand_dtype);
-  // Workspace: [tile R x C] [gx accumulator R x dim f32, only with several column tiles] [state].
-  const uint64_t tile_bytes = (R * C * esz + 255) & ~255ull;
+  // The tile's row pitch is a multiple of 128 elements: the logits product stores whole vectors, the row kernels read
+  // them, and the gradients' rows end in zeros up to whole K steps of the input gradient's product, whatever the
+  // vocabulary (with 32003 columns at their own pitch every one of these passes went element by element: 3500 tokens,
+  // d = 512: CE_BEFORE us for the loss, CE_AFTER with the pitch).
+  const uint64_t ldt = (C + 127) / 128 * 128;
+  // Workspace: [tile R x ldt] [gx accumulator R x dim f32, only with several column tiles] [state].
+  const uint64_t tile_bytes = (R * ldt * esz + 255) & ~255ull;
   const uint64_t gxacc_bytes = (gx && !one_tile) ? ((R * dim * 4 + 255) & ~255ull) : 0;
   void* ws = nullptr;
   int32_t rc = omx_workspace(ctx, tile_bytes + gxacc_bytes + ce_scratch_bytes(rows), &ws);
@@ -643,14 +684,13 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
   auto logits_tile = [&](uint64_t r0, uint64_t nr, uint64_t c0, uint64_t nc) -> int32_t {
     // tile[nr, nc] = x[r0.., :] . W[c0.., :]^T
     return omx_gemm_impl(ctx, F_LINEAR_CE, xb + r0 * dim * esz, dim, 1, wb + c0 * dim * esz, 1, dim, operand_dtype,
-                         tile, operand_dtype, nc, nr, dim, nc, 0);
+                         tile, operand_dtype, ldt, nr, dim, nc, 0);
   };
   for (uint64_t r0 = 0; r0 < rows; r0 += R) {
     const uint64_t nr = (rows - r0) < R ? (rows - r0) : R;
     // The whole vocabulary in one tile, with gradients wanted: one kernel reads the logits once.
-    const bool fuse = ctx->ce_fused && one_tile && want_grads && vocab <= static_cast<uint64_t>(CE_FUSED_THREADS) * CE_FUSED_PACKS * (16 / esz) &&
-                      (operand_dtype == OMX_F32 ? ce_vector_ok<float>(tile, vocab, static_cast<unsigned>(vocab))
-                                                : ce_vector_ok<unsigned short>(tile, vocab, static_cast<unsigned>(vocab)));
+    const bool fuse = ctx->ce_fused && one_tile && want_grads && vocab >= 16 / esz &&
+                      vocab <= static_cast<uint64_t>(CE_FUSED_THREADS) * CE_FUSED_PACKS * (16 / esz);
     // Pass 1: row statistics over every vocabulary tile.
     for (uint64_t c0 = 0; c0 < vocab; c0 += C) {
       const uint64_t nc = (vocab - c0) < C ? (vocab - c0) : C;
@@ -664,7 +704,7 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
         const uint64_t packs = (nc * esz / 16 + CE_FUSED_THREADS - 1) / CE_FUSED_THREADS;
 #define CE_FUSED(T_, P_)                                                                                          \
   omx_launch_timed(ctx, ce_row_fused_kernel<T_, P_>, grid, block, 0, timer.start(), timer.stop(),                 \
-                   static_cast<T_*>(tile), nc, r0, static_cast<unsigned>(nc), tg, has_ignore, ignore_index, s.st, \
+                   static_cast<T_*>(tile), ldt, r0, static_cast<unsigned>(nc), static_cast<unsigned>(ldt), tg, has_ignore, ignore_index, s.st, \
                    s.valid, ctx->fault, tag)
 #define CE_FUSED_P(T_)                              \
   do {                                              \
@@ -682,10 +722,10 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
         continue;
       }
       if (operand_dtype == OMX_F32)
-        launch_stats<float>(ctx, tile, nc, r0, nr, static_cast<unsigned>(c0), static_cast<unsigned>(nc), tg, s.st,
+        launch_stats<float>(ctx, tile, ldt, r0, nr, static_cast<unsigned>(c0), static_cast<unsigned>(nc), tg, s.st,
                             c0 == 0, tag);
       else
-        launch_stats<unsigned short>(ctx, tile, nc, r0, nr, static_cast<unsigned>(c0), static_cast<unsigned>(nc), tg,
+        launch_stats<unsigned short>(ctx, tile, ldt, r0, nr, static_cast<unsigned>(c0), static_cast<unsigned>(nc), tg,
                                      s.st, c0 == 0, tag);
       OMX_LAUNCH_CHECK(ctx, "ce_tile_stats_kernel");
     }
@@ -693,6 +733,7 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
     // Pass 2: gradient tiles and their two products.
     for (uint64_t c0 = 0; c0 < vocab; c0 += C) {
       const uint64_t nc = (vocab - c0) < C ? (vocab - c0) : C;
+      const unsigned zero_to = static_cast<unsigned>((nc + 127) / 128 * 128);
       if (!one_tile) {
         rc = logits_tile(r0, nr, c0, nc);
         if (rc != OMX_OK) return rc;
@@ -700,28 +741,28 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
       if (fuse) {
         // the gradients are already in the tile
       } else if (operand_dtype == OMX_F32)
-        launch_grad<float, float>(ctx, tile, tile, nc, nc, r0, nr, static_cast<unsigned>(c0),
-                                  static_cast<unsigned>(nc), tg, has_ignore, ignore_index, s.st, s.valid);
+        launch_grad<float, float>(ctx, tile, tile, ldt, ldt, r0, nr, static_cast<unsigned>(c0),
+                                  static_cast<unsigned>(nc), zero_to, tg, has_ignore, ignore_index, s.st, s.valid);
       else
-        launch_grad<unsigned short, unsigned short>(ctx, tile, tile, nc, nc, r0, nr, static_cast<unsigned>(c0),
-                                                    static_cast<unsigned>(nc), tg, has_ignore, ignore_index, s.st,
+        launch_grad<unsigned short, unsigned short>(ctx, tile, tile, ldt, ldt, r0, nr, static_cast<unsigned>(c0),
+                                                    static_cast<unsigned>(nc), zero_to, tg, has_ignore, ignore_index, s.st,
                                                     s.valid);
       OMX_LAUNCH_CHECK(ctx, "ce_tile_grad_kernel");
       if (gx) {
         // gx[r0.., :] (+)= G[nr, nc] . W[c0.., :]
         if (one_tile) {
-          rc = omx_gemm_impl(ctx, F_LINEAR_CE, tile, nc, 1, wb + c0 * dim * esz, dim, 1, operand_dtype,
+          rc = omx_gemm_impl(ctx, F_LINEAR_CE, tile, ldt, 1, wb + c0 * dim * esz, dim, 1, operand_dtype,
                              static_cast<char*>(gx) + r0 * dim * omx_dtype_size(gx_dtype), gx_dtype, dim, nr, nc, dim,
-                             0);
+                             0, nullptr, nullptr, zero_to);
         } else {
-          rc = omx_gemm_impl(ctx, F_LINEAR_CE, tile, nc, 1, wb + c0 * dim * esz, dim, 1, operand_dtype, gxacc,
-                             OMX_F32, dim, nr, nc, dim, c0 != 0);
+          rc = omx_gemm_impl(ctx, F_LINEAR_CE, tile, ldt, 1, wb + c0 * dim * esz, dim, 1, operand_dtype, gxacc,
+                             OMX_F32, dim, nr, nc, dim, c0 != 0, nullptr, nullptr, zero_to);
         }
         if (rc != OMX_OK) return rc;
       }
       if (gw) {
         // gw[c0.., :] (+)= G^T[nc, nr] . x[r0.., :]
-        rc = omx_gemm_impl(ctx, F_LINEAR_CE, tile, 1, nc, xb + r0 * dim * esz, dim, 1, operand_dtype,
+        rc = omx_gemm_impl(ctx, F_LINEAR_CE, tile, 1, ldt, xb + r0 * dim * esz, dim, 1, operand_dtype,
                            static_cast<float*>(gw) + c0 * dim, OMX_F32, dim, nc, nr, dim, r0 != 0);
         if (rc != OMX_OK) return rc;
       }

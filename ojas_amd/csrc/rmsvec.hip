@@ -38,16 +38,18 @@ struct Raw4<unsigned short> {
   }
 };
 
-// All of a row's loads (the weight row too, up to 1024 columns) are issued before the first is used: with the
-// sum stored between one chunk's loads and the next chunk's, a row was NCH + 1 memory latencies in a chain,
-// which is all there is to a call of a few rows (1024 rows of 768: 6.5 -> 4.5 us with the launch).
-template <typename TX, typename TA, typename TY, int NCH>
+// TOGETHER: all of a row's loads (the weight row too, up to 1024 columns) are issued before the first is used. With the
+// sum stored between one chunk's loads and the next chunk's, a row is NCH + 1 memory latencies in a chain, which is
+// all there is to a call of a few rows (1024 rows of 768: 6.5 -> 4.5 us with the launch). Where several workgroups
+// wait for every place on the chip the chain is hidden, and loads spread over the row's life keep the memory busier:
+// 16384 rows of 768 inside a training step 27.4 us in that form, 29.4 with the loads together.
+template <typename TX, typename TA, typename TY, int NCH, bool TOGETHER>
 __global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __restrict__ x, const TA* __restrict__ add,
                                                                  const float* __restrict__ w,
                                                                  float* __restrict__ sum_out, TY* __restrict__ y,
                                                                  size_t rows, int dim, float eps, OmxFaultWord* fault,
                                                                  unsigned long long tag) {
-  constexpr bool EARLY_W = NCH <= 4;
+  constexpr bool EARLY_W = TOGETHER && NCH <= 4;
   const int lane = threadIdx.x & 63;
   const size_t row = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -55,8 +57,7 @@ __global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __res
   Raw4<TX> xr[NCH];
   Raw4<TA> ar[NCH];
   Raw4<float> wr[EARLY_W ? NCH : 1];
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
+  auto load = [&](int j) {
     const int c = j * 256 + lane * 4;
     if (c < dim) {
       xr[j].load(x + base + c);
@@ -66,12 +67,17 @@ __global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __res
       xr[j].clear();
       ar[j].clear();
     }
+  };
+  if constexpr (TOGETHER) {
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) load(j);
   }
   float xv[NCH][4];
   float ss = 0.0f;
   bool bad = false;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
+    if constexpr (!TOGETHER) load(j);
     xr[j].get(xv[j]);
     if (add) {
       float av[4];
@@ -81,6 +87,7 @@ __global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __res
         xv[j][e] = xv[j][e] + av[e];
         bad |= !dev_finite(xv[j][e]);
       }
+      if (j * 256 + lane * 4 < dim) dev_store4<float>(sum_out, base + j * 256 + lane * 4, xv[j]);
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss += xv[j][e] * xv[j][e];
@@ -96,7 +103,6 @@ __global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __res
       float wv[4], out[4];
       if constexpr (EARLY_W) wr[j].get(wv);
       else dev_load4<float>(w, c, wv);
-      if (add) dev_store4<float>(sum_out, base + c, xv[j]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         out[e] = xv[j][e] * rstd * wv[e];
@@ -288,8 +294,10 @@ int32_t omx_rms_forward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const 
   const auto width = [](int32_t dtype) { return dtype == OMX_BF16 ? 2.0 : 4.0; };
   OmxKernelTimer timer(ctx, OMX_K_RMS_FWD, static_cast<double>(rows) * static_cast<double>(dim) *
                                                (width(x_dtype) + (add ? width(add_dtype) + 4.0 : 0.0) + width(y_dtype)));
+  // Up to half the waves the chip holds (32 per compute unit), nothing else hides a row's latencies.
+  const bool together = rows <= 16ull * static_cast<uint64_t>(ctx->cu_count > 0 ? ctx->cu_count : 256);
 #define RV_FWD(TX, TA, TY, N)                                                                                      \
-  omx_launch_timed(ctx, rms_fwd_vec_kernel<TX, TA, TY, N>, grid, block, 0, timer.start(), timer.stop(),            \
+  omx_launch_timed(ctx, together ? rms_fwd_vec_kernel<TX, TA, TY, N, true> : rms_fwd_vec_kernel<TX, TA, TY, N, false>, grid, block, 0, timer.start(), timer.stop(),            \
                    static_cast<const TX*>(x), static_cast<const TA*>(add), w, sum_out, static_cast<TY*>(y),        \
                    static_cast<size_t>(rows), static_cast<int>(dim), eps, ctx->fault, tag)
 #define RV_FWD_N(TX, TA, TY)      \

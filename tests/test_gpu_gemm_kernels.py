@@ -239,6 +239,27 @@ def test_strided_batch_of_weight_gradients(be, mode, rows, kin, nout, layers):
         assert err <= 1e-5 * max(1.0, float(np.max(np.abs(ogw)))), (l, err)
 
 
+@pytest.mark.parametrize("mode", [1, 3, 4, 9, 10])
+@pytest.mark.parametrize("tokens,m,n,pitch", [(65, 264, 256, 264), (127, 257, 192, 264), (191, 250, 384, 256), (1, 256, 256, 256),
+                                              (3500, 512, 768, 512), (4161, 1000, 1152, 1000), (6300, 2048, 2304, 2048)])
+def test_reductions_of_any_length_end_inside_a_step(be, mode, tokens, m, n, pitch):
+    """Weight gradients over a number of tokens that no K step divides: the rows behind the last token (NaN here) are
+    never multiplied, nor are the columns between a row's end and its pitch."""
+    from ojas_amd.backend import BF16
+
+    print(f"gemm ragged K mode {mode} {m}x{n} over {tokens}", flush=True)
+    be.set_option("gemm_dma", mode)
+    rng = np.random.default_rng(tokens + mode)
+    gy = np.full((tokens + 256, pitch), np.nan, np.float32)
+    x = np.full((tokens + 256, n), np.nan, np.float32)
+    gy[:tokens, :m] = orc.round_bf16((rng.standard_normal((tokens, m)) * 0.5).astype(np.float32).ravel()).reshape(tokens, m)
+    x[:tokens] = orc.round_bf16((rng.standard_normal((tokens, n)) * 0.5).astype(np.float32).ravel()).reshape(tokens, n)
+    want = gy[:tokens, :m].T @ x[:tokens]
+    got = be.download(be.gemm(be.upload(gy, BF16), (1, pitch), be.upload(x, BF16), (n, 1), m, tokens, n))
+    be.set_option("gemm_dma", 1)
+    assert float(np.max(np.abs(got - want))) <= 2e-5 * max(1.0, float(np.max(np.abs(want))))
+
+
 @pytest.mark.parametrize("rows,kin,nout,layers", [(4096, 16, 512, 6), (4096, 384, 48, 5), (2048, 8, 256, 16)])
 def test_strided_batch_of_thin_weight_gradients_splits_the_reduction(be, rows, kin, nout, layers):
     """A batch of thin outputs over a long reduction (an adapter's rank x d gradients over the

@@ -325,6 +325,39 @@ def test_linear_cross_entropy_one_read_kernel_agrees_with_the_two_kernels(be, bf
     close(got[1][2], ogw, tol, "one-read gw")
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,dim,vocab,chunk_cols", [(2100, 512, 1003, 1003), (2100, 512, 1003, 520), (40, 64, 7, 7),
+                                                       (40, 64, 3, 3), (33, 64, 129, 129), (600, 128, 4097, 4097)])
+def test_linear_cross_entropy_of_odd_vocabularies(be, dtype, rows, dim, vocab, chunk_cols):
+    """Vocabularies that no vector and no K step divides: the logits rows have padding, which takes part in nothing."""
+    from ojas_amd.backend import BF16, F32
+
+    print(f"linear CE {dtype} {rows}x{dim} vocab {vocab} by {chunk_cols}", flush=True)
+    rng = np.random.default_rng(rows + vocab)
+    bf = dtype == "bf16"
+    rnd = (lambda a: orc.round_bf16(a.ravel()).reshape(a.shape)) if bf else (lambda a: a)
+    x = rnd((rng.standard_normal((rows, dim)) * 0.5).astype(np.float32))
+    w = rnd((rng.standard_normal((vocab, dim)) * 0.1).astype(np.float32))
+    targets = rng.integers(0, vocab, rows).astype(np.uint32)
+    targets[:2] = vocab - 1
+    up = (lambda a: be.upload(a, BF16)) if bf else be.upload
+    loss, gx, gw = be.linear_cross_entropy_mean(up(x), up(w), be.upload(targets), 2, (rows, chunk_cols))
+    logits = x.astype(np.float64) @ w.astype(np.float64).T
+    keep = targets != 2
+    p = np.exp(logits - logits.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    want = -np.log(p[np.arange(rows), targets])[keep].mean()
+    g = p
+    g[np.arange(rows), targets] -= 1.0
+    g[~keep] = 0.0
+    g /= keep.sum()
+    tol = 2e-2 if bf else 1e-4
+    assert abs(float(be.download(loss)[0]) - want) <= (1e-3 if bf else 1e-5) * abs(want)
+    for name, got, ref in (("gx", gx, g @ w), ("gw", gw, g.T @ x)):
+        err = float(np.max(np.abs(be.download_f32(got) - ref)))
+        assert err <= tol * float(np.max(np.abs(ref))), (name, err)
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("poison", ["nan", "+inf", "-inf"])
 @pytest.mark.parametrize("as_target", [False, True])
