@@ -482,7 +482,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   if (operand_dtype == OMX_F32 && ctx->gemm_dma_mode == 1 && !(epi && epi->mode != OMX_EPI_NONE))
     frag32 = omx_gemm_frag32_tile(ctx, g, a_km, b_km);
   int dma_variant = -1;
-  if (!thin && !skinny && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km)) {
+  if (!thin && !skinny && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) {
     const int mode = ctx->gemm_dma_mode;
     if (mode == 1 && ctx->gemm_forced_tiling >= 0) {
       dma_variant = ctx->gemm_forced_tiling;

@@ -273,7 +273,7 @@ __device__ __forceinline__ bool gemm_store_block(const GemmArgs& g, int split, c
 // bf16 kernels with direct-to-LDS loads and a 256 x 256 (variant 9), 256 x 128 (variant 3) or
 // 128 x 128 (variant 6) workgroup tile. Needs 16-byte aligned operands, and whole K steps in the
 // rows of k-contiguous ones.
-bool omx_gemm_dma_eligible(const GemmArgs& g, bool a_km, bool b_km);
+bool omx_gemm_dma_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain);
 bool omx_gemm_w4_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain);
 void omx_gemm_dma_tile(int variant, int* bm, int* bn);
 int32_t omx_gemm_dma_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int variant);

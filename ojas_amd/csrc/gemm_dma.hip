@@ -44,8 +44,8 @@ static bool whole_steps(const GemmArgs& g, bool a_km, bool b_km, int step) {
   return b_km && (a_km || g.a_k >= up) && up <= 0x7fffffffl;
 }
 
-bool omx_gemm_dma_eligible(const GemmArgs& g, bool a_km, bool b_km) {
-  if (!whole_steps(g, a_km, b_km, 64) || !g.a_vec || !g.b_vec) return false;
+bool omx_gemm_dma_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain) {
+  if (!whole_steps(g, a_km, b_km, 64) || (g.K % 64 != 0 && !plain) || !g.a_vec || !g.b_vec) return false;
   if (g.lda >= (1l << 22) || g.ldb >= (1l << 22)) return false;  // a tile's lane offsets are 32 bits of bytes
   return true;
 }

@@ -7,11 +7,9 @@
 
 namespace {
 
-// EPI: the store pass this instantiation is compiled for (OMX_EPI_*), or OMX_EPI_ANY for the one
-// that chooses at run time. A kernel of its own per store pass keeps each one's code (a few KiB of
-// straight-line stores) and registers out of the others.
-constexpr int OMX_EPI_ANY = -1;
-template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI = OMX_EPI_ANY>
+// EPI: the store pass (OMX_EPI_*). A kernel of its own per store pass keeps each one's code (a few KiB of
+// straight-line stores) and registers out of the others. TAIL: see StepBase.
+template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI, bool TAIL = false>
 __global__ __launch_bounds__(WGM* WGN * 64, dma_waves_per_simd(WGM* WGN, NST*(WGM* TM + WGN * TN) * 32 * DBK * 2)) void
 gemm_dma_kernel(GemmArgs g) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -78,8 +76,8 @@ gemm_dma_kernel(GemmArgs g) {
   // Everything a K step needs is computed here, once per tile: the loads' global addresses and
   // the fragments' LDS offsets. Inside the loop the stage is a compile-time constant (the loop
   // body is unrolled over the stages), so a step is loads, LDS reads and MFMAs and little else.
-  TileLoadsOff<A_KM, BM, DBK, NW> la;
-  TileLoadsOff<B_KM, BN, DBK, NW> lb;
+  TileLoadsOff<A_KM, BM, DBK, NW, TAIL> la;
+  TileLoadsOff<B_KM, BN, DBK, NW, TAIL> lb;
   la.init(A, g.lda, m0, g.M, ks_begin * DBK, g.k_rows, wave, lane);
   lb.init(B, g.ldb, n0, g.N, ks_begin * DBK, g.k_rows, wave, lane);
   const unsigned lds0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem)));
@@ -200,8 +198,8 @@ gemm_dma_kernel(GemmArgs g) {
     bool stored = false;
     if constexpr (kFastStores) {
       const bool interior = grow0 + 32 <= g.M && gcol0 + TN * 32 <= g.N;
-      if constexpr (EPI == OMX_EPI_ANY || EPI == OMX_EPI_NONE) {
-        if (interior && g.epi == OMX_EPI_NONE && (g.splits > 1 ? (g.N & 3) == 0 : g.c_vec != 0)) {
+      if constexpr (EPI == OMX_EPI_NONE) {
+        if (interior && (g.splits > 1 ? (g.N & 3) == 0 : g.c_vec != 0)) {
           if (g.splits > 1) bad |= gemm_store_block<0, PPR>(g, split, cs, CPW, grow0, gcol0, lane);
           else if (g.c_bf16) bad |= gemm_store_block<1, PPR>(g, split, cs, CPW, grow0, gcol0, lane);
           else if (!g.accumulate) bad |= gemm_store_block<2, PPR>(g, split, cs, CPW, grow0, gcol0, lane);
@@ -209,20 +207,7 @@ gemm_dma_kernel(GemmArgs g) {
           stored = true;
         }
       }
-      if constexpr (EPI == OMX_EPI_ANY) {
-        if (!stored && interior && g.epi != OMX_EPI_NONE && g.c_vec != 0) {
-          if (g.epi == OMX_EPI_GELU_FWD) {
-            bad |= g.epi_tanh ? gemm_epilogue_block<OMX_EPI_GELU_FWD, true, PPR>(g, cs, CPW, grow0, gcol0, lane)
-                              : gemm_epilogue_block<OMX_EPI_GELU_FWD, false, PPR>(g, cs, CPW, grow0, gcol0, lane);
-          } else if (g.epi == OMX_EPI_AXPBY) {
-            bad |= gemm_epilogue_block<OMX_EPI_AXPBY, false, PPR>(g, cs, CPW, grow0, gcol0, lane);
-          } else {
-            bad |= g.epi_tanh ? gemm_epilogue_block<OMX_EPI_GELU_BWD, true, PPR>(g, cs, CPW, grow0, gcol0, lane)
-                              : gemm_epilogue_block<OMX_EPI_GELU_BWD, false, PPR>(g, cs, CPW, grow0, gcol0, lane);
-          }
-          stored = true;
-        }
-      } else if constexpr (EPI == OMX_EPI_AXPBY) {
+      if constexpr (EPI == OMX_EPI_AXPBY) {
         if (interior && g.c_vec != 0) {
           bad |= gemm_epilogue_block<OMX_EPI_AXPBY, false, PPR>(g, cs, CPW, grow0, gcol0, lane);
           stored = true;
@@ -257,13 +242,14 @@ template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int N
 int32_t launch_dma(omx_ctx* ctx, const GemmArgs& g) {
   constexpr int BM = WGM * TM * 32, BN = WGN * TN * 32;
   constexpr int smem = NST * (BM + BN) * DBK * 2;
-  auto kernel = &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST>;
-  // The two tiles the dispatcher picks by itself have a kernel per store pass.
-  if constexpr (DBK == 32 && TM * TN <= 4 && NST == 3) {
-    kernel = g.epi == OMX_EPI_GELU_FWD   ? &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_GELU_FWD>
-             : g.epi == OMX_EPI_GELU_BWD ? &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_GELU_BWD>
-             : g.epi == OMX_EPI_AXPBY    ? &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_AXPBY>
-                                         : &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_NONE>;
+  // A kernel per store pass.
+  auto kernel = g.epi == OMX_EPI_GELU_FWD   ? &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_GELU_FWD>
+                : g.epi == OMX_EPI_GELU_BWD ? &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_GELU_BWD>
+                : g.epi == OMX_EPI_AXPBY    ? &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_AXPBY>
+                                            : &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_NONE>;
+  // (gemm_dma.hip takes a ragged reduction only with the plain store pass)
+  if constexpr (B_KM) {
+    if (g.k_rows != g.K) kernel = &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_NONE, true>;
   }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    smem));

@@ -27,25 +27,24 @@ __device__ __forceinline__ void static_for(F&& f) {
 // Where a wave's direct-to-LDS loads of one operand tile start: a wave-uniform address of the tile's first element at
 // the current K step, beside which every lane and load has a 32-bit byte offset that never changes. A K step advances
 // scalars only (64-bit vector additions would take issue slots from the matrix instructions).
-// K rows: a k-major operand ends after `rows_left` more K rows, wherever in a step that is. Its loads are buffer loads
-// bounded to what is left of the current step, and lanes past the bound write zeros into LDS, so a reduction of any
-// length (weight gradients: K = tokens) runs whole steps. It costs three scalar instructions per step; the register-
-// staged kernel that such lengths took before ran a 512 x 2048 x 6 gradient over 3500 tokens in 225 us, this one in
-// DMA_TAIL_US. A k-contiguous operand's rows have to hold whole steps.
-template <bool KM>
-struct StepBase;
-template <>
-struct StepBase<false> {
+// TAIL: a k-major operand ends after `rows_left` more K rows, wherever in a step that is. Its loads are then buffer
+// loads bounded to what is left of the current step, and lanes past the bound write zeros into LDS, so a reduction of
+// any length (weight gradients: K = tokens) runs whole steps. Six products of 512 x 2048 over 3500 rows: 225 us on the
+// register-staged kernel, which such lengths took before, 69 us here. A kernel of its own, because the bounded loads
+// cost 1 % where no step is ragged (2635 -> 2662 us over the weight gradients of 12 layers of d = 768). A k-contiguous
+// operand's rows have to hold whole steps.
+template <bool KM, bool TAIL>
+struct StepBase {
   const char* at;
   long step;  // bytes between consecutive K steps
   __device__ __forceinline__ void init(const void* p, long ld, int row0, int k0, int /*k_rows*/, int bk) {
-    const unsigned long long addr =
-        reinterpret_cast<unsigned long long>(p) + static_cast<unsigned long long>(static_cast<long>(row0) * ld + k0) * 2;
+    const long first = KM ? static_cast<long>(k0) * ld + row0 : static_cast<long>(row0) * ld + k0;
+    const unsigned long long addr = reinterpret_cast<unsigned long long>(p) + static_cast<unsigned long long>(first) * 2;
     // (tile coordinates come out of vector divisions: back to scalars)
     const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(addr));
     const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(addr >> 32));
     at = reinterpret_cast<const char*>((static_cast<unsigned long long>(hi) << 32) | lo);
-    step = bk * 2;
+    step = (KM ? bk * ld : bk) * 2;
   }
   __device__ __forceinline__ void advance() { at += step; }
   // 16 bytes per lane into LDS at `lds` + IMM + 16 * lane. Written as assembly: the compiler cannot tell that this
@@ -58,7 +57,7 @@ struct StepBase<false> {
   }
 };
 template <>
-struct StepBase<true> {
+struct StepBase<true, true> {
   unsigned long long at;
   u32x4 rsrc;      // base address (48 bits, no stride), bytes from it, 32-bit raw data
   int rows_left;   // K rows from this step on
@@ -99,13 +98,13 @@ struct StepBase<true> {
 // offset, so edge tiles take this form too (a k-major operand's last 16-byte chunk may reach past its last column into
 // the padding of the row, which is at least 16 bytes aligned; those values only meet outputs that are not stored).
 // Needs 255 rows of the leading dimension to fit 32 bits of bytes.
-template <bool KM, int ROWS, int BK, int NW>
+template <bool KM, int ROWS, int BK, int NW, bool TAIL = false>
 struct TileLoadsOff {
   static constexpr int TOTAL = ROWS * BK * 2 / 1024;
   static constexpr int N = TOTAL / NW;
   static_assert(TOTAL % NW == 0, "the same number of loads in every wave");
   unsigned off[N];
-  StepBase<KM> base;
+  StepBase<KM, TAIL> base;
 
   // `k_rows`: where the K rows of a k-major operand end.
   __device__ __forceinline__ void init(const unsigned short* __restrict__ p, long ld, int row0, int rows, int k0,

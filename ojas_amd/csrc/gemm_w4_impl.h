@@ -44,11 +44,11 @@ __device__ __forceinline__ int w4_km_swizzle(int kr) {
 }
 
 // Loads of one operand (see StepBase for the base address and the end of the K rows).
-template <bool KM, int ROWS>
+template <bool KM, int ROWS, bool TAIL>
 struct W4Loads {
   static constexpr int N = ROWS / 32;  // ROWS / 8 loads of 1 KiB per step, four waves
   unsigned off[N];
-  StepBase<KM> base;
+  StepBase<KM, TAIL> base;
   __device__ __forceinline__ void init(const unsigned short* __restrict__ p, long ld, int row0, int rows, int k0,
                                        int k_rows, int wave, int lane) {
 #pragma unroll
@@ -121,7 +121,7 @@ struct W4Frags {
   }
 };
 
-template <bool A_KM, bool B_KM, int TN>
+template <bool A_KM, bool B_KM, int TN, bool TAIL>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   static_assert(!A_KM || B_KM, "a k-major A goes with a k-major B");
   static_assert(TN == 4 || TN == 3, "256 x 256 or 256 x 192 tiles");
@@ -178,8 +178,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   const int ks_begin = split * g.ksteps_per_split;
   const int ks_end = min(g.K / W4_BK, ks_begin + g.ksteps_per_split);
   const int steps = ks_end - ks_begin;
-  W4Loads<A_KM, W4_BM> la;
-  W4Loads<B_KM, W4_BN> lb;
+  W4Loads<A_KM, W4_BM, TAIL> la;
+  W4Loads<B_KM, W4_BN, TAIL> lb;
   la.init(A, g.lda, m0, g.M, ks_begin * W4_BK, g.k_rows, wave, lane);
   lb.init(B, g.ldb, n0, g.N, ks_begin * W4_BK, g.k_rows, wave, lane);
   const unsigned lds_wave =
@@ -502,7 +502,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
 
 template <bool A_KM, bool B_KM, int TN>
 int32_t launch_w4(omx_ctx* ctx, const GemmArgs& g) {
-  auto kernel = &gemm_w4_kernel<A_KM, B_KM, TN>;
+  auto kernel = &gemm_w4_kernel<A_KM, B_KM, TN, false>;
+  if constexpr (B_KM) {
+    if (g.k_rows != g.K) kernel = &gemm_w4_kernel<A_KM, B_KM, TN, true>;
+  }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    W4_SMEM));
   omx_launch_timed(ctx, kernel, dim3(g.tiles_m * g.tiles_n * g.splits, g.batches), dim3(256), W4_SMEM, ctx->timing_start,

