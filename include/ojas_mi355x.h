@@ -400,6 +400,11 @@ int32_t omx_adamw_step_bounded(omx_ctx* ctx, void* param_f32, const void* grad_f
                                void* moment1_f32, void* moment2_f32, uint64_t n, uint64_t step,
                                const omx_adamw_config* config, void* param_bf16,
                                int32_t inputs_bounded, void* unbounded_flag);
+/* omx_adamw_step on `count` tensors in one set of launches (a small model's tens of vectors), bit for bit what
+ * a call for each gives: each tensor is all-or-nothing by itself. The arrays hold device pointers. */
+int32_t omx_adamw_step_batched(omx_ctx* ctx, void* const* params_f32, const void* const* grads_f32,
+                               void* const* moments1_f32, void* const* moments2_f32, const uint64_t* lens,
+                               uint64_t count, uint64_t step, const omx_adamw_config* config);
 /* ojas_core::MuonNs5Config (backend.rs:548-570). */
 typedef struct {
   double lr, momentum, weight_decay;
@@ -436,6 +441,9 @@ int32_t omx_residual_add(omx_ctx* ctx, const void* x, int32_t x_dtype, const voi
                          void* out, int32_t out_dtype, uint64_t n);
 /* BackendFloat::accumulate_grad / scale_grad (backend.rs:1473-1510). */
 int32_t omx_accumulate_grad(omx_ctx* ctx, void* acc_f32, const void* grad_f32, uint64_t n);
+/* omx_accumulate_grad on `count` pairs in one launch. */
+int32_t omx_accumulate_grads(omx_ctx* ctx, void* const* accs_f32, const void* const* grads_f32, const uint64_t* lens,
+                             uint64_t count);
 int32_t omx_scale_grad(omx_ctx* ctx, void* grad_f32, float scale, uint64_t n);
 /* BackendFloat::gelu_erf_* / gelu_tanh_* (backend.rs:1175-1220). tanh_form
  * selects the tanh approximation. */

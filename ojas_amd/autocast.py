@@ -145,6 +145,11 @@ class Autocast:
         self.inner.accumulate_grad(acc, grad)
         self._wrote(acc)
 
+    def accumulate_grads(self, accs, grads):
+        self.inner.accumulate_grads(accs, grads)
+        for acc in accs:
+            self._wrote(acc)
+
     def scale_grad(self, grad, scale):
         self.inner.scale_grad(grad, scale)
         self._wrote(grad)
@@ -157,4 +162,14 @@ class Autocast:
     def muon_ns5_step(self, param, grad, momentum, *args, **kwargs):
         self.inner.muon_ns5_step(param, grad, momentum, *args, **kwargs)
         for t in (param, momentum):
+            self._wrote(t)
+
+    def adamw_step_batched(self, params, grads, m1, m2, *args, **kwargs):
+        self.inner.adamw_step_batched(params, grads, m1, m2, *args, **kwargs)
+        for t in (*params, *m1, *m2):
+            self._wrote(t)
+
+    def muon_ns5_step_batched(self, params, grads, momenta, *args, **kwargs):
+        self.inner.muon_ns5_step_batched(params, grads, momenta, *args, **kwargs)
+        for t in (*params, *momenta):
             self._wrote(t)

@@ -555,6 +555,25 @@ class MiBackend:
         _native.omx_adamw_step_bounded(self._context, param, grad, moment1, moment2, param.numel, step,
                                        C.addressof(config), param_bf16, (1 if inputs_bounded else 0), unbounded_flag)
 
+    def adamw_step_batched(self, params, grads, moments1, moments2, step: int, config: AdamWConfig):
+        """`adamw_step` on several tensors in one set of launches (in place, each all-or-nothing by itself)."""
+        lists = (params, grads, moments1, moments2)
+        for p, g, m1, m2 in zip(*lists):
+            shapes.adamw_step_dims(p, g, m1, m2)
+        if len({len(ts) for ts in lists}) != 1:
+            raise OjasError(SHAPE, "adamw_step_batched: one gradient and two moments for each parameter")
+        tables = [self._pointers(ts) for ts in lists]
+        _native.omx_adamw_step_batched(self._context, *[C.addressof(t) for t in tables],
+                                       C.addressof(lens := self._lengths(params)), len(params), step, C.addressof(config))
+
+    @staticmethod
+    def _pointers(ts):
+        return (C.c_void_p * max(len(ts), 1))(*[t.ptr for t in ts])
+
+    @staticmethod
+    def _lengths(ts):
+        return (C.c_uint64 * max(len(ts), 1))(*[t.numel for t in ts])
+
     def muon_ns5_step(self, param, grad, momentum, config: MuonNs5Config, param_bf16=None):
         rows, cols = param.shape
         _native.omx_muon_ns5_step(self._context, param, grad, momentum, rows, cols, C.addressof(config),
@@ -573,11 +592,10 @@ class MiBackend:
                                           C.addressof(config))
 
     def clip_grad_norm(self, grads: Sequence[DeviceTensor], max_norm: float) -> float:
-        n = len(grads)
-        ptrs = (C.c_void_p * max(n, 1))(*[g.ptr for g in grads])
-        lens = (C.c_uint64 * max(n, 1))(*[g.numel for g in grads])
+        ptrs, lens = self._pointers(grads), self._lengths(grads)
         norm = C.c_float()
-        _native.omx_clip_grad_norm(self._context, C.addressof(ptrs), C.addressof(lens), n, max_norm, C.addressof(norm))
+        _native.omx_clip_grad_norm(self._context, C.addressof(ptrs), C.addressof(lens), len(grads), max_norm,
+                                   C.addressof(norm))
         return float(norm.value)
 
     # ---- elementwise / layout ----
@@ -591,6 +609,14 @@ class MiBackend:
 
     def accumulate_grad(self, acc, grad):
         _native.omx_accumulate_grad(self._context, acc, grad, acc.numel)
+
+    def accumulate_grads(self, accs, grads):
+        """`accumulate_grad` on several pairs in one launch."""
+        if len(accs) != len(grads) or any(a.numel != g.numel for a, g in zip(accs, grads)):
+            raise OjasError(SHAPE, "accumulate_grads: one gradient of the same size for each accumulator")
+        tables = self._pointers(accs), self._pointers(grads)
+        _native.omx_accumulate_grads(self._context, *[C.addressof(t) for t in tables],
+                                     C.addressof(lens := self._lengths(accs)), len(accs))
 
     def scale_grad(self, grad, scale: float):
         _native.omx_scale_grad(self._context, grad, scale, grad.numel)

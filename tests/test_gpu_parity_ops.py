@@ -325,6 +325,54 @@ def test_linear_cross_entropy_one_read_kernel_agrees_with_the_two_kernels(be, bf
     close(got[1][2], ogw, tol, "one-read gw")
 
 
+@pytest.mark.parametrize("count", [1, 47, 48, 49, 100])
+def test_lists_of_tensors_equal_a_call_for_each(be, count):
+    """AdamW and accumulation on lists (48 tensors to a launch) give the bits of a call for each tensor, whatever the
+    lengths and alignments; a tensor with a value that is not finite keeps its parameter and moments and no other's."""
+    from ojas_amd.backend import AdamWConfig, DeviceTensor, OjasError
+
+    print(f"tensor lists {count}", flush=True)
+    rng = np.random.default_rng(count)
+    lens = [int(n) for n in rng.choice([1, 3, 4, 5, 1023, 1024, 1025, 4099, 70000], count)]
+    host = [[rng.standard_normal(n).astype(np.float32) for n in lens] for _ in range(4)]
+    host[3] = [np.abs(v) for v in host[3]]
+    if count > 1:
+        host[1][count // 2][-1] = np.float32(3e38)  # g^2 overflows: that tensor is refused
+
+    def upload(a, odd):
+        whole = be.upload(np.concatenate([np.zeros(int(odd), np.float32), a]))
+        return whole, DeviceTensor(be, whole.ptr + 4 * int(odd), a.shape, whole.dtype, owns=False)
+
+    def copies():
+        kept = [[upload(a, i % 3 == 1) for i, a in enumerate(ts)] for ts in host]
+        return kept, [[v for _, v in ts] for ts in kept]
+
+    cfg = AdamWConfig(1e-2, 0.9, 0.95, 1e-8, 0.1)
+    keep1, (p1, g1, m1, v1) = copies()
+    keep2, (p2, g2, m2, v2) = copies()
+    for args in zip(p1, g1, m1, v1):
+        be.adamw_step(*args, 3, cfg)
+    be.adamw_step_batched(p2, g2, m2, v2, 3, cfg)
+    if count > 1:
+        with pytest.raises(OjasError):
+            be.sync()
+    for one, many in zip((p1, m1, v1), (p2, m2, v2)):
+        for a, b in zip(one, many):
+            assert np.array_equal(be.download(a), be.download(b))
+    for a, b in zip(p1, m1):
+        be.accumulate_grad(a, b)
+    be.accumulate_grads(p2, m2)
+    for a, b, h in zip(p1, p2, host[0]):
+        assert np.array_equal(be.download(a), be.download(b))
+    norm = be.clip_grad_norm(p2, 0.5)
+    before = [be.download(a) for a in p1]
+    want = float(np.sqrt(sum(float(np.sum(a.astype(np.float64) ** 2)) for a in before)))
+    assert abs(norm - want) <= 1e-6 * want
+    coef = np.float32(np.float32(0.5) / (np.float32(norm) + np.float32(1e-6)))
+    for a, b in zip(before, p2):
+        assert np.array_equal(be.download(b), a * min(coef, np.float32(1)))
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("rows,dim,vocab,chunk_cols", [(2100, 512, 1003, 1003), (2100, 512, 1003, 520), (40, 64, 7, 7),
                                                        (40, 64, 3, 3), (33, 64, 129, 129), (600, 128, 4097, 4097)])
