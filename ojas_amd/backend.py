@@ -88,7 +88,7 @@ def load_library() -> C.CDLL:
     return lib
 
 
-class MiBackend:
+class MiBackend(_native.Methods):
     """`impl Backend for MiBackend`: BackendId::Hip, Numerics::Fast, bf16 operands accepted."""
 
     id = "hip"
@@ -1020,3 +1020,7 @@ def _clip_shape_first(method):
 for _name, (_validator, _operands) in _VALIDATED.items():
     setattr(MiBackend, _name, _shape_first(_name, getattr(MiBackend, _name), _validator, _operands))
 MiBackend.clip_grad_norm = _clip_shape_first(MiBackend.clip_grad_norm)
+# The methods that exist in native code too: the well-formed call goes there, what it does not take comes back here.
+for _name in [n for n in vars(_native.Methods) if not n.startswith("_")]:
+    setattr(MiBackend, "_checked_" + _name, vars(MiBackend)[_name])
+    delattr(MiBackend, _name)

@@ -376,12 +376,12 @@ int32_t check_unary(omx_ctx* ctx, const char* op, int32_t dtype, uint64_t n, std
   do {                                                                                                  \
     if ((dtype) == OMX_F32) {                                                                           \
       typedef float T_;                                                                                 \
-      if (vec) hipLaunchKernelGGL((KERNEL<T_, 4>), grid, dim3(BK_THREADS), 0, ctx->stream, __VA_ARGS__); \
-      else hipLaunchKernelGGL((KERNEL<T_, 1>), grid, dim3(BK_THREADS), 0, ctx->stream, __VA_ARGS__);    \
+      if (vec) omx_launch(ctx, (KERNEL<T_, 4>), grid, dim3(BK_THREADS), 0, __VA_ARGS__); \
+      else omx_launch(ctx, (KERNEL<T_, 1>), grid, dim3(BK_THREADS), 0, __VA_ARGS__);    \
     } else {                                                                                            \
       typedef unsigned short T_;                                                                        \
-      if (vec) hipLaunchKernelGGL((KERNEL<T_, 4>), grid, dim3(BK_THREADS), 0, ctx->stream, __VA_ARGS__); \
-      else hipLaunchKernelGGL((KERNEL<T_, 1>), grid, dim3(BK_THREADS), 0, ctx->stream, __VA_ARGS__);    \
+      if (vec) omx_launch(ctx, (KERNEL<T_, 4>), grid, dim3(BK_THREADS), 0, __VA_ARGS__); \
+      else omx_launch(ctx, (KERNEL<T_, 1>), grid, dim3(BK_THREADS), 0, __VA_ARGS__);    \
     }                                                                                                   \
   } while (0)
 
@@ -402,7 +402,7 @@ int32_t launch_rope(omx_ctx* ctx, const char* op, uint32_t fault_op, const void*
   unsigned long long tag = omx_tag(ctx, fault_op);
   dim3 grid = pack_grid(rows * (half / v));
 #define ROPE_K(T_, V_)                                                                                           \
-  hipLaunchKernelGGL((rope_kernel<T_, V_, BACKWARD>), grid, dim3(BK_THREADS), 0, ctx->stream,                    \
+  omx_launch(ctx, (rope_kernel<T_, V_, BACKWARD>), grid, dim3(BK_THREADS), 0,                    \
                      static_cast<const T_*>(x), static_cast<const float*>(cos), static_cast<const float*>(sin), \
                      static_cast<T_*>(y), static_cast<size_t>(rows), static_cast<int>(dim),                      \
                      static_cast<size_t>(time), static_cast<size_t>(heads), ctx->fault, tag)
@@ -437,7 +437,7 @@ int32_t compute_gates(omx_ctx* ctx, uint32_t fault_op, const void* input, const 
   int32_t rc = omx_gemm_impl(ctx, fault_op, input, d_model, 1, weight, 1, d_model, operand_dtype, gates, OMX_F32, heads,
                              rows, d_model, heads, 0);
   if (rc != OMX_OK) return rc;
-  hipLaunchKernelGGL(gate_sigmoid_kernel, pack_grid(rows * heads), dim3(BK_THREADS), 0, ctx->stream, gates,
+  omx_launch(ctx, gate_sigmoid_kernel, pack_grid(rows * heads), dim3(BK_THREADS), 0, gates,
                      static_cast<const float*>(bias), static_cast<size_t>(rows * heads), static_cast<int>(heads),
                      ctx->fault, omx_tag(ctx, fault_op));
   OMX_LAUNCH_CHECK(ctx, "gate_sigmoid_kernel");
@@ -615,7 +615,7 @@ int32_t omx_per_head_sigmoid_gate_forward(omx_ctx* ctx, const void* input, const
   unsigned long long tag = omx_tag(ctx, F_GATE_FORWARD);
   dim3 grid = pack_grid(packs);
 #define GATE_APPLY(TA, TY, V_)                                                                                    \
-  hipLaunchKernelGGL((gate_apply_kernel<TA, TY, V_>), grid, dim3(BK_THREADS), 0, ctx->stream,                     \
+  omx_launch(ctx, (gate_apply_kernel<TA, TY, V_>), grid, dim3(BK_THREADS), 0,                     \
                      static_cast<const TA*>(attn), gates, static_cast<TY*>(y), packs, head_packs, ctx->fault, tag)
   typedef unsigned short h16;
   const int key = (attn_dtype == OMX_BF16 ? 2 : 0) | (y_dtype == OMX_BF16 ? 1 : 0);
@@ -691,7 +691,7 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
   unsigned long long tag = omx_tag(ctx, F_GATE_BACKWARD);
   dim3 grid(static_cast<unsigned>(blocks));
 #define GATE_BWD(TA, TO, TZ, V_)                                                                                 \
-  hipLaunchKernelGGL((gate_bwd_kernel<TA, TA, TO, TZ, V_>), grid, dim3(BK_THREADS), lds_bytes, ctx->stream,      \
+  omx_launch(ctx, (gate_bwd_kernel<TA, TA, TO, TZ, V_>), grid, dim3(BK_THREADS), lds_bytes,      \
                      static_cast<const TA*>(attn), static_cast<const TA*>(gy), gates, static_cast<TO*>(g_attn),  \
                      static_cast<TZ*>(gz), partial, static_cast<size_t>(rows), static_cast<int>(heads),          \
                      head_packs, group, block_rows, ctx->fault, tag)
@@ -775,7 +775,7 @@ int32_t omx_per_head_sigmoid_gate_input_grad_add(omx_ctx* ctx, const void* gz, c
     const unsigned long long tag = omx_tag(ctx, F_GATE_BACKWARD);
     dim3 grid(static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block));
 #define GATE_JOIN(TA_)                                                                                        \
-  hipLaunchKernelGGL(gate_input_grad_add_kernel<TA_>, grid, dim3(threads), 0, ctx->stream,                    \
+  omx_launch(ctx, gate_input_grad_add_kernel<TA_>, grid, dim3(threads), 0,                    \
                      static_cast<const unsigned short*>(gz), static_cast<const unsigned short*>(weight),      \
                      static_cast<const TA_*>(add_in), static_cast<float*>(out), rows, static_cast<int>(d_model), \
                      static_cast<int>(heads), rows_per_block, ctx->fault, tag)
@@ -826,7 +826,7 @@ int32_t omx_value_residual_blend_backward(omx_ctx* ctx, const void* value, const
             static_cast<const T_*>(gy), static_cast<const float*>(lambda), static_cast<T_*>(g_value),
             static_cast<T_*>(g_value0), partial, packs, ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "vres_bwd_kernel");
-  hipLaunchKernelGGL(vres_lambda_kernel, dim3(1), dim3(BK_THREADS), 0, ctx->stream, partial, static_cast<int>(grid.x),
+  omx_launch(ctx, vres_lambda_kernel, dim3(1), dim3(BK_THREADS), 0, partial, static_cast<int>(grid.x),
                      static_cast<const float*>(lambda), static_cast<float*>(g_lambda), ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "vres_lambda_kernel");
   return OMX_OK;

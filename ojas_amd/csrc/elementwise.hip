@@ -139,10 +139,10 @@ int32_t omx_convert(omx_ctx* ctx, const void* src, int32_t src_dtype, void* dst,
   if (n == 0) return OMX_OK;
   dim3 grid = ew_grid(n), block(EW_THREADS);
   if (src_dtype == OMX_F32 && dst_dtype == OMX_BF16)
-    hipLaunchKernelGGL((convert_kernel<float, unsigned short>), grid, block, 0, ctx->stream,
+    omx_launch(ctx, (convert_kernel<float, unsigned short>), grid, block, 0,
                        static_cast<const float*>(src), static_cast<unsigned short*>(dst), n);
   else if (src_dtype == OMX_BF16 && dst_dtype == OMX_F32)
-    hipLaunchKernelGGL((convert_kernel<unsigned short, float>), grid, block, 0, ctx->stream,
+    omx_launch(ctx, (convert_kernel<unsigned short, float>), grid, block, 0,
                        static_cast<const unsigned short*>(src), static_cast<float*>(dst), n);
   else if (src_dtype == dst_dtype)
     return omx_copy(ctx, dst, src, n * omx_dtype_size(src_dtype));
@@ -161,7 +161,7 @@ int32_t omx_fill_zero(omx_ctx* ctx, void* dst, uint64_t bytes) {
   if (reinterpret_cast<uintptr_t>(dst) & 3u) return omx_fail(ctx, OMX_SHAPE, "fill_zero: pointer not 4-byte aligned");
   uint64_t words = bytes / 4;
   int tail = static_cast<int>(bytes % 4);
-  hipLaunchKernelGGL(fill_zero_kernel, ew_grid(words), dim3(EW_THREADS), 0, ctx->stream,
+  omx_launch(ctx, fill_zero_kernel, ew_grid(words), dim3(EW_THREADS), 0,
                      static_cast<unsigned int*>(dst), words, static_cast<unsigned char*>(dst) + words * 4, tail);
   OMX_LAUNCH_CHECK(ctx, "fill_zero_kernel");
   return OMX_OK;
@@ -171,7 +171,7 @@ int32_t omx_cast_bf16(omx_ctx* ctx, const void* x, void* y, uint64_t n) {
   OMX_REQUIRE_CTX(ctx);
   if (!x || !y) return omx_fail(ctx, OMX_PLACEMENT, "cast_bf16: null device pointer");
   if (n == 0) return omx_fail(ctx, OMX_SHAPE, "cast_bf16: zero-sized axis");
-  hipLaunchKernelGGL(round_bf16_kernel, ew_grid(n), dim3(EW_THREADS), 0, ctx->stream, static_cast<const float*>(x),
+  omx_launch(ctx, round_bf16_kernel, ew_grid(n), dim3(EW_THREADS), 0, static_cast<const float*>(x),
                      static_cast<float*>(y), n);
   OMX_LAUNCH_CHECK(ctx, "round_bf16_kernel");
   return OMX_OK;
@@ -199,7 +199,7 @@ int32_t omx_residual_add(omx_ctx* ctx, const void* x, int32_t x_dtype, const voi
   unsigned long long tag = omx_tag(ctx, F_RESIDUAL_ADD);
   dim3 grid = ew_grid(n), block(EW_THREADS);
 #define ADD_K(TX, TY, TO)                                                                                   \
-  hipLaunchKernelGGL((add_kernel<TX, TY, TO>), grid, block, 0, ctx->stream, static_cast<const TX*>(x),      \
+  omx_launch(ctx, (add_kernel<TX, TY, TO>), grid, block, 0, static_cast<const TX*>(x),      \
                      static_cast<const TY*>(y), static_cast<TO*>(out), n, ctx->fault, tag)
   typedef unsigned short h16;
   const int key = (x_dtype == OMX_BF16 ? 4 : 0) | (y_dtype == OMX_BF16 ? 2 : 0) | (out_dtype == OMX_BF16 ? 1 : 0);
@@ -222,7 +222,7 @@ int32_t omx_accumulate_grad(omx_ctx* ctx, void* acc, const void* grad, uint64_t 
   OMX_REQUIRE_CTX(ctx);
   if (!acc || !grad) return omx_fail(ctx, OMX_PLACEMENT, "accumulate_grad: null device pointer");
   if (n == 0) return omx_fail(ctx, OMX_SHAPE, "accumulate_grad: zero-sized axis");
-  hipLaunchKernelGGL(accumulate_kernel, ew_grid(n), dim3(EW_THREADS), 0, ctx->stream, static_cast<float*>(acc),
+  omx_launch(ctx, accumulate_kernel, ew_grid(n), dim3(EW_THREADS), 0, static_cast<float*>(acc),
                      static_cast<const float*>(grad), n, ctx->fault, omx_tag(ctx, F_ACCUMULATE));
   OMX_LAUNCH_CHECK(ctx, "accumulate_kernel");
   return OMX_OK;
@@ -234,7 +234,7 @@ int32_t omx_scale_grad(omx_ctx* ctx, void* grad, float scale, uint64_t n) {
   if (n == 0) return omx_fail(ctx, OMX_SHAPE, "scale_grad: zero-sized axis");
   if (!(scale == scale) || scale == INFINITY || scale == -INFINITY)
     return omx_fail(ctx, OMX_NON_FINITE, "scale_grad");
-  hipLaunchKernelGGL(scale_kernel, ew_grid(n), dim3(EW_THREADS), 0, ctx->stream, static_cast<float*>(grad), scale, n,
+  omx_launch(ctx, scale_kernel, ew_grid(n), dim3(EW_THREADS), 0, static_cast<float*>(grad), scale, n,
                      ctx->fault, omx_tag(ctx, F_SCALE_GRAD));
   OMX_LAUNCH_CHECK(ctx, "scale_kernel");
   return OMX_OK;
@@ -249,7 +249,7 @@ int32_t omx_gelu_forward(omx_ctx* ctx, const void* x, void* y, int32_t dtype, ui
   unsigned long long tag = omx_tag(ctx, F_GELU_FORWARD);
   dim3 grid = ew_grid(n), block(EW_THREADS);
 #define GELU_FWD(T, TANH)                                                                                       \
-  hipLaunchKernelGGL((gelu_fwd_kernel<T, TANH>), grid, block, 0, ctx->stream, static_cast<const T*>(x), \
+  omx_launch(ctx, (gelu_fwd_kernel<T, TANH>), grid, block, 0, static_cast<const T*>(x), \
                      static_cast<T*>(y), n, ctx->fault, tag)
   if (dtype == OMX_F32) {
     if (tanh_form) GELU_FWD(float, true);
@@ -273,7 +273,7 @@ int32_t omx_gelu_backward(omx_ctx* ctx, const void* x, const void* gy, void* gx,
   unsigned long long tag = omx_tag(ctx, F_GELU_BACKWARD);
   dim3 grid = ew_grid(n), block(EW_THREADS);
 #define GELU_BWD(T, TANH)                                                                                       \
-  hipLaunchKernelGGL((gelu_bwd_kernel<T, TANH>), grid, block, 0, ctx->stream, static_cast<const T*>(x), \
+  omx_launch(ctx, (gelu_bwd_kernel<T, TANH>), grid, block, 0, static_cast<const T*>(x), \
                      static_cast<const T*>(gy), static_cast<T*>(gx), n, ctx->fault, tag)
   if (dtype == OMX_F32) {
     if (tanh_form) GELU_BWD(float, true);
@@ -298,14 +298,12 @@ int32_t omx_permute_0213(omx_ctx* ctx, const void* x, void* y, int32_t dtype, ui
   bool al16 = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0;
   if (row_bytes % 16 == 0 && al16) {
     size_t d3v = row_bytes / 16;
-    hipLaunchKernelGGL((permute_0213_kernel<uint4>), ew_grid(d0 * d1 * d2 * d3v), dim3(EW_THREADS), 0, ctx->stream,
+    omx_launch(ctx, (permute_0213_kernel<uint4>), ew_grid(d0 * d1 * d2 * d3v), dim3(EW_THREADS), 0,
                        static_cast<const uint4*>(x), static_cast<uint4*>(y), d0, d1, d2, d3v);
   } else if (esz == 4) {
-    hipLaunchKernelGGL((permute_0213_kernel<unsigned int>), ew_grid(d0 * d1 * d2 * d3), dim3(EW_THREADS), 0,
-                       ctx->stream, static_cast<const unsigned int*>(x), static_cast<unsigned int*>(y), d0, d1, d2, d3);
+    omx_launch(ctx, (permute_0213_kernel<unsigned int>), ew_grid(d0 * d1 * d2 * d3), dim3(EW_THREADS), 0, static_cast<const unsigned int*>(x), static_cast<unsigned int*>(y), d0, d1, d2, d3);
   } else {
-    hipLaunchKernelGGL((permute_0213_kernel<unsigned short>), ew_grid(d0 * d1 * d2 * d3), dim3(EW_THREADS), 0,
-                       ctx->stream, static_cast<const unsigned short*>(x), static_cast<unsigned short*>(y), d0, d1, d2,
+    omx_launch(ctx, (permute_0213_kernel<unsigned short>), ew_grid(d0 * d1 * d2 * d3), dim3(EW_THREADS), 0, static_cast<const unsigned short*>(x), static_cast<unsigned short*>(y), d0, d1, d2,
                        d3);
   }
   OMX_LAUNCH_CHECK(ctx, "permute_0213_kernel");
@@ -338,11 +336,11 @@ int32_t omx_token_windows(omx_ctx* ctx, const void* tokens, int32_t bytes_per_to
   const uint64_t n = batch * seq_len;
   const unsigned blocks = static_cast<unsigned>(std::min<uint64_t>((n + 255) / 256, 4096));
   if (bytes_per_token == 2)
-    hipLaunchKernelGGL((token_windows_kernel<unsigned short>), dim3(blocks), dim3(256), 0, ctx->stream,
+    omx_launch(ctx, (token_windows_kernel<unsigned short>), dim3(blocks), dim3(256), 0,
                        static_cast<const unsigned short*>(tokens), static_cast<const unsigned long long*>(ws),
                        static_cast<unsigned int*>(x), static_cast<unsigned int*>(y), batch, seq_len);
   else
-    hipLaunchKernelGGL((token_windows_kernel<unsigned int>), dim3(blocks), dim3(256), 0, ctx->stream,
+    omx_launch(ctx, (token_windows_kernel<unsigned int>), dim3(blocks), dim3(256), 0,
                        static_cast<const unsigned int*>(tokens), static_cast<const unsigned long long*>(ws),
                        static_cast<unsigned int*>(x), static_cast<unsigned int*>(y), batch, seq_len);
   OMX_LAUNCH_CHECK(ctx, "token_windows_kernel");

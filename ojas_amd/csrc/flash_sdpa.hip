@@ -1048,7 +1048,7 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
   dim3 kv_grid((s.kv_single ? blocks : pairs) * kv_planes);
   dim3 q_grid((s.q_single ? blocks : pairs) * q_planes);
   auto go = [&](auto dq_kernel, auto dkv_kernel, auto* gq_ptr, auto* gk_ptr, auto* gv_ptr) {
-    hipLaunchKernelGGL(dq_kernel, q_grid, block, 0, ctx->stream, q, k, v, out, resid, lse, delta, key_mean, gy, gq_ptr, s,
+    omx_launch(ctx, dq_kernel, q_grid, block, 0, q, k, v, out, resid, lse, delta, key_mean, gy, gq_ptr, s,
                        ctx->fault, tag);
     omx_launch_timed(ctx, dkv_kernel, kv_grid, block, 0, nullptr, timer.stop(), q, k, v, lse, delta, gy, gk_ptr, gv_ptr, s,
                      ctx->fault, tag);

@@ -548,7 +548,7 @@ int32_t omx_pack_i8_group(omx_ctx* ctx, const void* codes_i8, const void* scales
   const float* src_s = static_cast<const float*>(unpack ? blocked_scales : scales_f32);
   signed char* dst = static_cast<signed char*>(unpack ? const_cast<void*>(codes_i8) : blocked_codes);
   float* dst_s = static_cast<float*>(unpack ? const_cast<void*>(scales_f32) : blocked_scales);
-  hipLaunchKernelGGL(q8_pack_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, ctx->stream, src,
+  omx_launch(ctx, q8_pack_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, src,
                      src_s, dst, dst_s, static_cast<long>(nout), static_cast<long>(kin), unpack);
   OMX_LAUNCH_CHECK(ctx, "q8_pack_kernel");
   return OMX_OK;

@@ -540,13 +540,13 @@ template <typename T, int VEC>
 int32_t launch_kv_write(omx_ctx* ctx, const KvWrite& w) {
   const unsigned blocks = static_cast<unsigned>(std::min<size_t>((w.n / VEC + 255) / 256, 8192));
   if (w.n <= KV_ONE_LAUNCH) {
-    hipLaunchKernelGGL((kv_scan_write_kernel<T, VEC>), dim3((blocks + 3) / 4), dim3(KV_SCAN_THREADS), 0, ctx->stream, w);
+    omx_launch(ctx, (kv_scan_write_kernel<T, VEC>), dim3((blocks + 3) / 4), dim3(KV_SCAN_THREADS), 0, w);
     OMX_LAUNCH_CHECK(ctx, "kv_scan_write_kernel");
     return OMX_OK;
   }
-  hipLaunchKernelGGL((kv_scan_kernel<VEC>), dim3(blocks), dim3(256), 0, ctx->stream, w);
+  omx_launch(ctx, (kv_scan_kernel<VEC>), dim3(blocks), dim3(256), 0, w);
   OMX_LAUNCH_CHECK(ctx, "kv_scan_kernel");
-  hipLaunchKernelGGL((kv_write_kernel<T, VEC>), dim3(blocks), dim3(256), 0, ctx->stream, w);
+  omx_launch(ctx, (kv_write_kernel<T, VEC>), dim3(blocks), dim3(256), 0, w);
   OMX_LAUNCH_CHECK(ctx, "kv_write_kernel");
   return OMX_OK;
 }
@@ -554,7 +554,7 @@ int32_t launch_kv_write(omx_ctx* ctx, const KvWrite& w) {
 template <typename T, int LPK, int NPL>
 int32_t launch_group(omx_ctx* ctx, const KvArgs& a, dim3 grid, long rows_total, int waves) {
   auto go = [&](auto eight, auto four, auto one) {
-    hipLaunchKernelGGL((waves == 8 ? eight : waves == 4 ? four : one), grid, dim3(waves * 64), 0, ctx->stream, a);
+    omx_launch(ctx, (waves == 8 ? eight : waves == 4 ? four : one), grid, dim3(waves * 64), 0, a);
   };
   if (a.tq * a.group == 1)
     go(&cached_attention_group_kernel<T, LPK, 8, 1>, &cached_attention_group_kernel<T, LPK, 4, 1>,
@@ -564,8 +564,7 @@ int32_t launch_group(omx_ctx* ctx, const KvArgs& a, dim3 grid, long rows_total, 
        &cached_attention_group_kernel<T, LPK, 1, KG_ROWS>);
   OMX_LAUNCH_CHECK(ctx, "cached_attention_group_kernel");
   if (a.nparts == 1) return OMX_OK;
-  hipLaunchKernelGGL((cached_attention_merge_kernel<NPL>), dim3(static_cast<unsigned>(rows_total)), dim3(64), 0,
-                     ctx->stream, a, rows_total);
+  omx_launch(ctx, (cached_attention_merge_kernel<NPL>), dim3(static_cast<unsigned>(rows_total)), dim3(64), 0, a, rows_total);
   OMX_LAUNCH_CHECK(ctx, "cached_attention_merge_kernel");
   return OMX_OK;
 }
@@ -576,9 +575,9 @@ int32_t launch_attention(omx_ctx* ctx, const KvArgs& a, dim3 grid, size_t lds_by
     if (lds_bytes > 64 * 1024)  // beyond the default limit: ask for it (cheap, and idempotent)
       OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
-    hipLaunchKernelGGL(kernel, grid, dim3(64), lds_bytes, ctx->stream, a);
+    omx_launch(ctx, kernel, grid, dim3(64), lds_bytes, a);
     OMX_LAUNCH_CHECK(ctx, "cached_attention_partial_kernel");
-    hipLaunchKernelGGL(merge, dim3(static_cast<unsigned>(rows_total)), dim3(64), 0, ctx->stream, a, rows_total);
+    omx_launch(ctx, merge, dim3(static_cast<unsigned>(rows_total)), dim3(64), 0, a, rows_total);
     OMX_LAUNCH_CHECK(ctx, "cached_attention_merge_kernel");
     return OMX_OK;
   };

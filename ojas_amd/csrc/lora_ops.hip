@@ -246,7 +246,7 @@ int32_t omx_rope_half_split_inplace(omx_ctx* ctx, void* x, int32_t dtype, uint64
   if (tokens > 0x7fffffffull || heads * dim > 0x7fffffffull)
     return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: axis does not fit in i32", op);
   const long total = static_cast<long>(tokens * heads * (dim / 16));
-  hipLaunchKernelGGL(rope_pitched_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, ctx->stream,
+  omx_launch(ctx, rope_pitched_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
                      static_cast<unsigned short*>(x), static_cast<long>(pitch), static_cast<const float*>(cos_f32),
                      static_cast<const float*>(sin_f32), static_cast<long>(tokens), static_cast<int>(time),
                      static_cast<int>(heads), static_cast<int>(dim), backward ? -1.0f : 1.0f, ctx->fault,
@@ -275,13 +275,13 @@ int32_t omx_rope_half_split_pitched(omx_ctx* ctx, const void* x, int32_t x_dtype
   const dim3 grid(static_cast<unsigned>((total + 255) / 256));
   const unsigned long long tag = omx_tag(ctx, F_ROPE_FORWARD);
   if (x_dtype == OMX_BF16)
-    hipLaunchKernelGGL(rope_pitched_out_kernel<unsigned short>, grid, dim3(256), 0, ctx->stream,
+    omx_launch(ctx, rope_pitched_out_kernel<unsigned short>, grid, dim3(256), 0,
                        static_cast<const unsigned short*>(x), static_cast<unsigned short*>(out), static_cast<long>(pitch),
                        static_cast<const float*>(cos_f32), static_cast<const float*>(sin_f32), static_cast<long>(tokens),
                        static_cast<int>(time), static_cast<int>(heads), static_cast<int>(plain_heads),
                        static_cast<int>(dim), ctx->fault, tag);
   else
-    hipLaunchKernelGGL(rope_pitched_out_kernel<float>, grid, dim3(256), 0, ctx->stream, static_cast<const float*>(x),
+    omx_launch(ctx, rope_pitched_out_kernel<float>, grid, dim3(256), 0, static_cast<const float*>(x),
                        static_cast<unsigned short*>(out), static_cast<long>(pitch), static_cast<const float*>(cos_f32),
                        static_cast<const float*>(sin_f32), static_cast<long>(tokens), static_cast<int>(time),
                        static_cast<int>(heads), static_cast<int>(plain_heads), static_cast<int>(dim), ctx->fault, tag);
@@ -297,10 +297,10 @@ int32_t omx_init_normal(omx_ctx* ctx, void* dst, int32_t dtype, uint64_t n, uint
   const long pairs = static_cast<long>((n + 1) / 2);
   dim3 grid(static_cast<unsigned>((pairs + 255) / 256)), block(256);
   if (dtype == OMX_F32)
-    hipLaunchKernelGGL(init_normal_kernel<float>, grid, block, 0, ctx->stream, static_cast<float*>(dst),
+    omx_launch(ctx, init_normal_kernel<float>, grid, block, 0, static_cast<float*>(dst),
                        static_cast<long>(n), static_cast<unsigned long long>(seed), std);
   else
-    hipLaunchKernelGGL(init_normal_kernel<unsigned short>, grid, block, 0, ctx->stream,
+    omx_launch(ctx, init_normal_kernel<unsigned short>, grid, block, 0,
                        static_cast<unsigned short*>(dst), static_cast<long>(n), static_cast<unsigned long long>(seed), std);
   OMX_LAUNCH_CHECK(ctx, "init_normal_kernel");
   return OMX_OK;
@@ -315,8 +315,7 @@ int32_t omx_init_normal_i8_group(omx_ctx* ctx, void* codes_i8, void* scales_f32,
   if (nout == 0 || kin == 0 || kin % 32 != 0) return omx_fail(ctx, OMX_SHAPE, "%s: k_in must be a positive multiple of 32", op);
   if (!aligned16(codes_i8)) return omx_fail(ctx, OMX_SHAPE, "%s: codes must be 16-byte aligned", op);
   const long groups = static_cast<long>(nout * (kin / 32));
-  hipLaunchKernelGGL(init_normal_i8_group_kernel, dim3(static_cast<unsigned>((groups + 255) / 256)), dim3(256), 0,
-                     ctx->stream, static_cast<signed char*>(codes_i8), static_cast<float*>(scales_f32), groups,
+  omx_launch(ctx, init_normal_i8_group_kernel, dim3(static_cast<unsigned>((groups + 255) / 256)), dim3(256), 0, static_cast<signed char*>(codes_i8), static_cast<float*>(scales_f32), groups,
                      static_cast<unsigned long long>(seed), std);
   OMX_LAUNCH_CHECK(ctx, "init_normal_i8_group_kernel");
   return OMX_OK;
@@ -334,12 +333,10 @@ int32_t omx_swiglu_forward(omx_ctx* ctx, const void* gate_up, void* out, int32_t
   const long total = static_cast<long>(rows * (hidden / 8));
   const unsigned long long tag = omx_tag(ctx, F_MUL_FORWARD);
   if (dtype == OMX_BF16)
-    hipLaunchKernelGGL(swiglu_fwd_kernel<unsigned short>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
-                       ctx->stream, static_cast<const unsigned short*>(gate_up), static_cast<unsigned short*>(out),
+    omx_launch(ctx, swiglu_fwd_kernel<unsigned short>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, static_cast<const unsigned short*>(gate_up), static_cast<unsigned short*>(out),
                        static_cast<long>(rows), static_cast<long>(hidden), ctx->fault, tag);
   else
-    hipLaunchKernelGGL(swiglu_fwd_kernel<float>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
-                       ctx->stream, static_cast<const float*>(gate_up), static_cast<unsigned short*>(out),
+    omx_launch(ctx, swiglu_fwd_kernel<float>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, static_cast<const float*>(gate_up), static_cast<unsigned short*>(out),
                        static_cast<long>(rows), static_cast<long>(hidden), ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "swiglu_fwd_kernel");
   return OMX_OK;
@@ -358,13 +355,11 @@ int32_t omx_swiglu_backward(omx_ctx* ctx, const void* gate_up, const void* gy, v
   const long total = static_cast<long>(rows * (hidden / 8));
   const unsigned long long tag = omx_tag(ctx, F_MUL_BACKWARD);
   if (dtype == OMX_BF16)
-    hipLaunchKernelGGL(swiglu_bwd_kernel<unsigned short>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
-                       ctx->stream, static_cast<const unsigned short*>(gate_up), static_cast<const unsigned short*>(gy),
+    omx_launch(ctx, swiglu_bwd_kernel<unsigned short>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, static_cast<const unsigned short*>(gate_up), static_cast<const unsigned short*>(gy),
                        static_cast<unsigned short*>(g_gate_up), static_cast<long>(rows), static_cast<long>(hidden),
                        ctx->fault, tag);
   else
-    hipLaunchKernelGGL(swiglu_bwd_kernel<float>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
-                       ctx->stream, static_cast<const float*>(gate_up), static_cast<const unsigned short*>(gy),
+    omx_launch(ctx, swiglu_bwd_kernel<float>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, static_cast<const float*>(gate_up), static_cast<const unsigned short*>(gy),
                        static_cast<unsigned short*>(g_gate_up), static_cast<long>(rows), static_cast<long>(hidden),
                        ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "swiglu_bwd_kernel");

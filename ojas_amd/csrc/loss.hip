@@ -470,10 +470,10 @@ void launch_stats(omx_ctx* ctx, const void* tile, size_t ld, size_t row0, size_t
                   unsigned int ncols, const unsigned int* targets, CeState st, int first, unsigned long long tag) {
   dim3 grid(static_cast<unsigned>(nrows)), block(CE_THREADS);
   if (ce_vector_ok<T>(tile, ld))
-    hipLaunchKernelGGL((ce_tile_stats_kernel<T, ce_vec<T>()>), grid, block, 0, ctx->stream,
+    omx_launch(ctx, (ce_tile_stats_kernel<T, ce_vec<T>()>), grid, block, 0,
                        static_cast<const T*>(tile), ld, row0, col0, ncols, targets, st, first, ctx->fault, tag);
   else
-    hipLaunchKernelGGL((ce_tile_stats_kernel<T, 1>), grid, block, 0, ctx->stream, static_cast<const T*>(tile), ld,
+    omx_launch(ctx, (ce_tile_stats_kernel<T, 1>), grid, block, 0, static_cast<const T*>(tile), ld,
                        row0, col0, ncols, targets, st, first, ctx->fault, tag);
 }
 template <typename TL, typename TG>
@@ -484,13 +484,13 @@ void launch_grad(omx_ctx* ctx, const void* tile, void* grad, size_t ld, size_t l
   // 16-byte packs on both sides need logits and gradients of one element size.
   if constexpr (sizeof(TL) == sizeof(TG)) {
     if (ce_vector_ok<TL>(tile, ld) && ce_vector_ok<TG>(grad, ld_grad)) {
-      hipLaunchKernelGGL((ce_tile_grad_kernel<TL, TG, ce_vec<TL>()>), grid, block, 0, ctx->stream,
+      omx_launch(ctx, (ce_tile_grad_kernel<TL, TG, ce_vec<TL>()>), grid, block, 0,
                          static_cast<const TL*>(tile), static_cast<TG*>(grad), ld, ld_grad, row0, col0, ncols, zero_to, targets,
                          has_ignore, ignore, st, valid);
       return;
     }
   }
-  hipLaunchKernelGGL((ce_tile_grad_kernel<TL, TG, 1>), grid, block, 0, ctx->stream, static_cast<const TL*>(tile),
+  omx_launch(ctx, (ce_tile_grad_kernel<TL, TG, 1>), grid, block, 0, static_cast<const TL*>(tile),
                      static_cast<TG*>(grad), ld, ld_grad, row0, col0, ncols, zero_to, targets, has_ignore, ignore, st, valid);
 }
 
@@ -514,8 +514,7 @@ int32_t count_valid(omx_ctx* ctx, const unsigned int* targets, uint64_t rows, ui
                     unsigned int ignore, unsigned int* valid, unsigned long long tag) {
   int32_t rc = omx_fill_zero(ctx, valid, 4);
   if (rc != OMX_OK) return rc;
-  hipLaunchKernelGGL(ce_count_valid_kernel, dim3(static_cast<unsigned>((rows + 255) / 256)), dim3(256), 0,
-                     ctx->stream, targets, rows, vocab, has_ignore, ignore, valid, ctx->fault, tag);
+  omx_launch(ctx, ce_count_valid_kernel, dim3(static_cast<unsigned>((rows + 255) / 256)), dim3(256), 0, targets, rows, vocab, has_ignore, ignore, valid, ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "ce_count_valid_kernel");
   return OMX_OK;
 }
@@ -543,7 +542,7 @@ int32_t ce_forward_in(omx_ctx* ctx, const void* logits, int32_t logits_dtype, co
   if (logits_dtype == OMX_F32) launch_stats<float>(ctx, logits, vocab, 0, rows, 0, vocab, tg, s.st, 1, tag);
   else launch_stats<unsigned short>(ctx, logits, vocab, 0, rows, 0, vocab, tg, s.st, 1, tag);
   OMX_LAUNCH_CHECK(ctx, "ce_tile_stats_kernel");
-  hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(1024), 0, ctx->stream, s.st, tg, rows, has_ignore, ignore_index,
+  omx_launch(ctx, ce_mean_kernel, dim3(1), dim3(1024), 0, s.st, tg, rows, has_ignore, ignore_index,
                      s.valid, static_cast<float*>(loss), ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "ce_mean_kernel");
   return OMX_OK;
@@ -620,7 +619,7 @@ int32_t omx_cross_entropy_mean_backward(omx_ctx* ctx, const void* logits, int32_
   else launch_stats<unsigned short>(ctx, logits, vocab, 0, rows, 0, vocab, tg, s.st, 1, tag);
   OMX_LAUNCH_CHECK(ctx, "ce_tile_stats_kernel");
   // The mean kernel also raises the all-ignored fault, as the forward does.
-  hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(1024), 0, ctx->stream, s.st, tg, rows, has_ignore, ignore_index,
+  omx_launch(ctx, ce_mean_kernel, dim3(1), dim3(1024), 0, s.st, tg, rows, has_ignore, ignore_index,
                      s.valid, loss_scratch, ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "ce_mean_kernel");
   if (logits_dtype == OMX_F32 && grad_dtype == OMX_F32)
@@ -773,7 +772,7 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
       if (rc != OMX_OK) return rc;
     }
   }
-  hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(1024), 0, ctx->stream, s.st, tg, rows, has_ignore, ignore_index,
+  omx_launch(ctx, ce_mean_kernel, dim3(1), dim3(1024), 0, s.st, tg, rows, has_ignore, ignore_index,
                      s.valid, static_cast<float*>(loss), ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "ce_mean_kernel");
   return OMX_OK;

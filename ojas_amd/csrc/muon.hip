@@ -242,10 +242,10 @@ int32_t run_muon(omx_ctx* ctx, const MuonTensors& t, unsigned count, uint64_t ro
   uint64_t x_off = L.x, xn_off = L.xn;
   const unsigned nb = static_cast<unsigned>((len + MU_BLOCK - 1) / MU_BLOCK);
   const dim3 block(MU_THREADS), over_len(mu_grid(len), count);
-  hipLaunchKernelGGL(muon_momentum_kernel, dim3(nb, count), block, 0, ctx->stream, t, w, len, s, ctx->fault, tag);
-  hipLaunchKernelGGL(muon_norm_kernel, dim3(1, count), dim3(1024), 0, ctx->stream, w, static_cast<size_t>(nb), s.bf16,
+  omx_launch(ctx, muon_momentum_kernel, dim3(nb, count), block, 0, t, w, len, s, ctx->fault, tag);
+  omx_launch(ctx, muon_norm_kernel, dim3(1, count), dim3(1024), 0, w, static_cast<size_t>(nb), s.bf16,
                      ctx->fault, tag);
-  hipLaunchKernelGGL((muon_normalize_kernel<TX>), over_len, block, 0, ctx->stream, w, x_off, len);
+  omx_launch(ctx, (muon_normalize_kernel<TX>), over_len, block, 0, w, x_off, len);
   OMX_LAUNCH_CHECK(ctx, "muon prologue");
   const bool tall = rows > cols;
   const uint64_t r = tall ? cols : rows, c = tall ? rows : cols;
@@ -271,7 +271,7 @@ int32_t run_muon(omx_ctx* ctx, const MuonTensors& t, unsigned count, uint64_t ro
     rc = omx_gemm_impl(ctx, F_MUON, am, r, 1, am, r, 1, XD, a2, XD, r, r, r, r, 0, fused ? &sum_b : nullptr, bp);
     if (rc != OMX_OK) return rc;
     if (!fused)
-      hipLaunchKernelGGL((muon_combine_b_kernel<TX>), dim3(mu_grid(r * r), count), block, 0, ctx->stream, w,
+      omx_launch(ctx, (muon_combine_b_kernel<TX>), dim3(mu_grid(r * r), count), block, 0, w,
                          static_cast<size_t>(r * r), s);
     // X_next = a X + B X, with BX in X's own physical layout: B X' when wide, X B^T when tall.
     const OmxGemmEpilogue sum_x{OMX_EPI_AXPBY, 0, x, nullptr, s.a, 1.0f};
@@ -280,14 +280,14 @@ int32_t run_muon(omx_ctx* ctx, const MuonTensors& t, unsigned count, uint64_t ro
     else rc = omx_gemm_impl(ctx, F_MUON, x, cols, 1, a2, 1, r, XD, xn, XD, cols, rows, cols, cols, 0, ex, bp);
     if (rc != OMX_OK) return rc;
     if (!fused)
-      hipLaunchKernelGGL((muon_combine_x_kernel<TX>), over_len, block, 0, ctx->stream, w, x_off, xn_off, len, s,
+      omx_launch(ctx, (muon_combine_x_kernel<TX>), over_len, block, 0, w, x_off, xn_off, len, s,
                          ctx->fault, tag);
     OMX_LAUNCH_CHECK(ctx, "muon newton-schulz step");
     std::swap(x_off, xn_off);
   }
-  hipLaunchKernelGGL((muon_check_update_kernel<TX>), over_len, block, 0, ctx->stream, t, w, x_off, len, s, ctx->fault,
+  omx_launch(ctx, (muon_check_update_kernel<TX>), over_len, block, 0, t, w, x_off, len, s, ctx->fault,
                      tag);
-  hipLaunchKernelGGL((muon_apply_kernel<TX>), over_len, block, 0, ctx->stream, t, w, x_off, len, s);
+  omx_launch(ctx, (muon_apply_kernel<TX>), over_len, block, 0, t, w, x_off, len, s);
   OMX_LAUNCH_CHECK(ctx, "muon apply");
   return OMX_OK;
 }

@@ -516,8 +516,8 @@ int32_t omx_adamw_step_batched(omx_ctx* ctx, void* const* params, const void* co
     }
     unsigned int* refuse = static_cast<unsigned int*>(ws) + t;
     const dim3 grid(list.spans.first[took]), block(OPT_THREADS);
-    hipLaunchKernelGGL(adamw_list_kernel<false>, grid, block, 0, ctx->stream, list, a, refuse, ctx->fault, omx_tag(ctx, F_ADAMW));
-    hipLaunchKernelGGL(adamw_list_kernel<true>, grid, block, 0, ctx->stream, list, a, refuse, ctx->fault, omx_tag(ctx, F_ADAMW));
+    omx_launch(ctx, adamw_list_kernel<false>, grid, block, 0, list, a, refuse, ctx->fault, omx_tag(ctx, F_ADAMW));
+    omx_launch(ctx, adamw_list_kernel<true>, grid, block, 0, list, a, refuse, ctx->fault, omx_tag(ctx, F_ADAMW));
     OMX_LAUNCH_CHECK(ctx, "adamw_list_kernel");
     t += took;
   }
@@ -540,7 +540,7 @@ int32_t omx_accumulate_grads(omx_ctx* ctx, void* const* accs, const void* const*
       list.acc[i] = static_cast<float*>(accs[t + i]);
       list.grad[i] = static_cast<const float*>(grads[t + i]);
     }
-    hipLaunchKernelGGL(accumulate_list_kernel, dim3(list.spans.first[took]), dim3(OPT_THREADS), 0, ctx->stream, list, ctx->fault,
+    omx_launch(ctx, accumulate_list_kernel, dim3(list.spans.first[took]), dim3(OPT_THREADS), 0, list, ctx->fault,
                        omx_tag(ctx, F_ACCUMULATE));
     OMX_LAUNCH_CHECK(ctx, "accumulate_list_kernel");
     t += took;
@@ -570,12 +570,12 @@ int32_t omx_clip_grad_norm(omx_ctx* ctx, void* const* grads, const uint64_t* len
     NormList list;
     const uint64_t took = fill_spans(list.spans, lens + t, count - t, NORM_BLOCK);
     for (uint64_t i = 0; i < took; ++i) list.x[i] = static_cast<const float*>(grads[t + i]);
-    hipLaunchKernelGGL(sumsq_list_kernel, dim3(list.spans.first[took]), dim3(OPT_THREADS), 0, ctx->stream, list, partial + at);
+    omx_launch(ctx, sumsq_list_kernel, dim3(list.spans.first[took]), dim3(OPT_THREADS), 0, list, partial + at);
     OMX_LAUNCH_CHECK(ctx, "sumsq_list_kernel");
     at += list.spans.first[took];
     t += took;
   }
-  hipLaunchKernelGGL(sumsq_final_kernel, dim3(1), dim3(1024), 0, ctx->stream, partial, blocks, total);
+  omx_launch(ctx, sumsq_final_kernel, dim3(1), dim3(1024), 0, partial, blocks, total);
   OMX_LAUNCH_CHECK(ctx, "sumsq_final_kernel");
   // The norm is a host value: this is the step's first sync point, and it
   // also reports any fault raised by the ops that produced the gradients.
@@ -595,7 +595,7 @@ int32_t omx_clip_grad_norm(omx_ctx* ctx, void* const* grads, const uint64_t* len
       ScaleList list;
       const uint64_t took = fill_spans(list.spans, lens + t, count - t, OPT_THREADS * 4);
       for (uint64_t i = 0; i < took; ++i) list.x[i] = static_cast<float*>(grads[t + i]);
-      hipLaunchKernelGGL(scale_list_kernel, dim3(list.spans.first[took]), dim3(OPT_THREADS), 0, ctx->stream, list, coef);
+      omx_launch(ctx, scale_list_kernel, dim3(list.spans.first[took]), dim3(OPT_THREADS), 0, list, coef);
       OMX_LAUNCH_CHECK(ctx, "scale_list_kernel");
       t += took;
     }

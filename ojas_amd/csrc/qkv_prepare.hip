@@ -310,8 +310,8 @@ int32_t omx_qkv_prepare_forward(omx_ctx* ctx, const void* qkv_lin, int32_t lin_d
   const uint64_t rows = tokens * (heads + 2 * kv_heads);
   const unsigned long long tag = omx_tag(ctx, F_RMS_FORWARD);
 #define QP_FWD(D_, LIN_)                                                                                           \
-  hipLaunchKernelGGL((qkv_prepare_fwd_kernel<D_, LIN_>), dim3(grid_for(ctx, rows, QP_THREADS / (D_ / 8))),             \
-                     dim3(QP_THREADS), 0, ctx->stream, static_cast<const LIN_*>(qkv_lin),                              \
+  omx_launch(ctx, (qkv_prepare_fwd_kernel<D_, LIN_>), dim3(grid_for(ctx, rows, QP_THREADS / (D_ / 8))),             \
+                     dim3(QP_THREADS), 0, static_cast<const LIN_*>(qkv_lin),                              \
                      static_cast<unsigned short*>(qkv_out), static_cast<const float*>(q_weight),                       \
                      static_cast<const float*>(k_weight), static_cast<const float*>(cos), static_cast<const float*>(sin), \
                      static_cast<const LIN_*>(value0), static_cast<const float*>(lambda), s, ctx->fault, tag)
@@ -361,7 +361,7 @@ int32_t omx_qkv_prepare_backward(omx_ctx* ctx, const void* qkv_lin, int32_t lin_
   float* partial_lambda = stage + OMX_COLUMN_SUM_GROUPS * 2 * head_dim;
   const unsigned long long tag = omx_tag(ctx, F_RMS_BACKWARD);
 #define QP_BWD(D_, LIN_)                                                                                               \
-  hipLaunchKernelGGL((qkv_prepare_bwd_kernel<D_, LIN_>), dim3(blocks), dim3(QP_THREADS), 0, ctx->stream,               \
+  omx_launch(ctx, (qkv_prepare_bwd_kernel<D_, LIN_>), dim3(blocks), dim3(QP_THREADS), 0,               \
                      static_cast<const LIN_*>(qkv_lin), static_cast<const unsigned short*>(g_qkv),                     \
                      static_cast<unsigned short*>(g_qkv_lin), static_cast<const float*>(q_weight),                     \
                      static_cast<const float*>(k_weight), static_cast<const float*>(cos), static_cast<const float*>(sin), \
@@ -385,7 +385,7 @@ int32_t omx_qkv_prepare_backward(omx_ctx* ctx, const void* qkv_lin, int32_t lin_
   rc = omx_copy(ctx, g_k_weight, summed + head_dim, head_dim * sizeof(float));
   if (rc != OMX_OK) return rc;
   if (value0) {
-    hipLaunchKernelGGL(qkv_lambda_kernel, dim3(1), dim3(256), 0, ctx->stream, partial_lambda, static_cast<int>(blocks),
+    omx_launch(ctx, qkv_lambda_kernel, dim3(1), dim3(256), 0, partial_lambda, static_cast<int>(blocks),
                        static_cast<const float*>(lambda), static_cast<float*>(g_lambda), ctx->fault, tag);
     OMX_LAUNCH_CHECK(ctx, "qkv_lambda_kernel");
   }

@@ -619,7 +619,7 @@ int32_t launch_rms_fwd(omx_ctx* ctx, const void* x, const float* w, void* y, uin
   int per = per_for_dim(dim);
 #define RMS_FWD(P)                                                                                              \
   case P:                                                                                                       \
-    hipLaunchKernelGGL((rms_fwd_kernel<TX, TY, P>), grid, block, 0, ctx->stream, static_cast<const TX*>(x), w, \
+    omx_launch(ctx, (rms_fwd_kernel<TX, TY, P>), grid, block, 0, static_cast<const TX*>(x), w, \
                        static_cast<TY*>(y), rows, static_cast<int>(dim), eps, ctx->fault, tag);                 \
     break;
   switch (per) {
@@ -649,7 +649,7 @@ int32_t launch_rms_bwd(omx_ctx* ctx, const void* x, const float* w, const void* 
   int per = per_for_dim(dim);
 #define RMS_BWD(P)                                                                                                  \
   case P:                                                                                                           \
-    hipLaunchKernelGGL((rms_bwd_kernel<TX, TG, TO, P>), grid, block, smem, ctx->stream, static_cast<const TX*>(x), \
+    omx_launch(ctx, (rms_bwd_kernel<TX, TG, TO, P>), grid, block, smem, static_cast<const TX*>(x), \
                        w, static_cast<const TG*>(gy), static_cast<TO*>(gx), static_cast<float*>(partial), rows,     \
                        static_cast<int>(dim), eps, rows_per_block, ctx->fault, tag);                                \
     break;
@@ -715,7 +715,7 @@ int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t 
   if (scratch && blocks > 4 * OMX_COLUMN_SUM_GROUPS) {
     // Stage 1: group g adds its contiguous share of the rows into scratch[g]; stage 2 adds the groups.
     const int per_group = static_cast<int>((blocks + OMX_COLUMN_SUM_GROUPS - 1) / OMX_COLUMN_SUM_GROUPS);
-    hipLaunchKernelGGL(column_sum_groups_kernel, dim3(col_blocks, OMX_COLUMN_SUM_GROUPS), dim3(256), 0, ctx->stream,
+    omx_launch(ctx, column_sum_groups_kernel, dim3(col_blocks, OMX_COLUMN_SUM_GROUPS), dim3(256), 0,
                        partial, scratch, static_cast<int>(blocks), static_cast<int>(dim), per_group);
     OMX_LAUNCH_CHECK(ctx, "column_sum_groups_kernel");
     partial = scratch;
@@ -802,7 +802,7 @@ int32_t omx_embedding_forward(omx_ctx* ctx, const void* table, int32_t table_dty
   dim3 grid(static_cast<unsigned>((tokens + 3) / 4)), block(ROW_THREADS);
   const unsigned int* idp = static_cast<const unsigned int*>(ids);
 #define EMB_FWD(TT, TO)                                                                                      \
-  hipLaunchKernelGGL((embedding_fwd_kernel<TT, TO>), grid, block, 0, ctx->stream, static_cast<const TT*>(table), \
+  omx_launch(ctx, (embedding_fwd_kernel<TT, TO>), grid, block, 0, static_cast<const TT*>(table), \
                      idp, static_cast<TO*>(out), tokens, vocab, static_cast<int>(dim), ctx->fault, tag)
   if (table_dtype == OMX_F32 && out_dtype == OMX_F32) EMB_FWD(float, float);
   else if (table_dtype == OMX_F32) EMB_FWD(float, unsigned short);
@@ -855,21 +855,21 @@ static int32_t embedding_backward_impl(omx_ctx* ctx, const void* ids, const void
   OMX_LAUNCH_CHECK(ctx, "count_ids_kernel");
   if (scan_blocks > 4 && scan_blocks <= SCAN_MAX_BLOCKS) {
     const dim3 sgrid(static_cast<unsigned>(scan_blocks));
-    hipLaunchKernelGGL(scan_totals_kernel, sgrid, dim3(1024), 0, ctx->stream, counts, scan_totals, vocab);
+    omx_launch(ctx, scan_totals_kernel, sgrid, dim3(1024), 0, counts, scan_totals, vocab);
     OMX_LAUNCH_CHECK(ctx, "scan_totals_kernel");
-    hipLaunchKernelGGL(scan_blocks_kernel, sgrid, dim3(1024), 0, ctx->stream, counts, scan_totals, offsets, cursor, vocab);
+    omx_launch(ctx, scan_blocks_kernel, sgrid, dim3(1024), 0, counts, scan_totals, offsets, cursor, vocab);
     OMX_LAUNCH_CHECK(ctx, "scan_blocks_kernel");
   } else {
-    hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(1024), 0, ctx->stream, counts, offsets, cursor, vocab);
+    omx_launch(ctx, scan_counts_kernel, dim3(1), dim3(1024), 0, counts, offsets, cursor, vocab);
     OMX_LAUNCH_CHECK(ctx, "scan_counts_kernel");
   }
-  hipLaunchKernelGGL(fill_positions_kernel, tgrid, dim3(256), 0, ctx->stream, idp, cursor, positions, tokens, vocab);
+  omx_launch(ctx, fill_positions_kernel, tgrid, dim3(256), 0, idp, cursor, positions, tokens, vocab);
   OMX_LAUNCH_CHECK(ctx, "fill_positions_kernel");
   dim3 vgrid(static_cast<unsigned>((vocab + 3) / 4));
-  hipLaunchKernelGGL(sort_short_segments_kernel, vgrid, dim3(ROW_THREADS), 0, ctx->stream, offsets, positions, sorted,
+  omx_launch(ctx, sort_short_segments_kernel, vgrid, dim3(ROW_THREADS), 0, offsets, positions, sorted,
                      long_count, long_rows, vocab);
   OMX_LAUNCH_CHECK(ctx, "sort_short_segments_kernel");
-  hipLaunchKernelGGL(sort_long_segments_kernel, dim3(256), dim3(1024), 0, ctx->stream, offsets, positions, sorted,
+  omx_launch(ctx, sort_long_segments_kernel, dim3(256), dim3(1024), 0, offsets, positions, sorted,
                      long_count, long_rows, tokens);
   OMX_LAUNCH_CHECK(ctx, "sort_long_segments_kernel");
   const bool vec4 = dim % 4 == 0 && (reinterpret_cast<uintptr_t>(grad) & 15u) == 0 &&
@@ -914,7 +914,7 @@ int32_t omx_argmax_rows(omx_ctx* ctx, const void* x, uint64_t rows, uint64_t col
   if (cols > 0xfffffffeull) return omx_fail(ctx, OMX_OUT_OF_RANGE, "argmax_rows: cols does not fit in u32");
   if (rows > 0x7fffffffull) return omx_fail(ctx, OMX_OUT_OF_RANGE, "argmax_rows: rows does not fit in i32");
   auto launch = [&](auto kernel, int threads) {
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(threads), 0, ctx->stream, static_cast<const float*>(x),
+    omx_launch(ctx, kernel, dim3(static_cast<unsigned>(rows)), dim3(threads), 0, static_cast<const float*>(x),
                        static_cast<unsigned int>(cols), static_cast<unsigned int*>(out), ctx->fault, omx_tag(ctx, F_ARGMAX));
   };
   // A quarter of a thousand columns feeds a wave; from four thousand on a row has work for sixteen.
@@ -933,7 +933,7 @@ int32_t omx_topk_rows(omx_ctx* ctx, const void* x, uint64_t rows, uint64_t cols,
   if (k == 0 || k > cols) return omx_fail(ctx, OMX_SHAPE, "topk_rows: k %llu outside 1..=%llu", (unsigned long long)k,
                                           (unsigned long long)cols);
   if (cols > 0xfffffffeull) return omx_fail(ctx, OMX_OUT_OF_RANGE, "topk_rows: cols does not fit in u32");
-  hipLaunchKernelGGL(topk_rows_kernel, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(ROW_THREADS), 0, ctx->stream,
+  omx_launch(ctx, topk_rows_kernel, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(ROW_THREADS), 0,
                      static_cast<const float*>(x), rows, static_cast<unsigned int>(cols), static_cast<unsigned int>(k),
                      static_cast<float*>(values), static_cast<unsigned int*>(ids), ctx->fault, omx_tag(ctx, F_TOPK));
   OMX_LAUNCH_CHECK(ctx, "topk_rows_kernel");

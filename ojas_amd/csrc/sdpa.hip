@@ -386,7 +386,7 @@ int32_t omx_causal_sdpa_forward(omx_ctx* ctx, const void* q, const void* k, cons
   const long rows = static_cast<long>(batch) * heads * time;
   dim3 grid(static_cast<unsigned>((rows + 3) / 4)), block(SD_THREADS);
 #define SDPA_FWD(TI, TO)                                                                                          \
-  hipLaunchKernelGGL((sdpa_fwd_rows_kernel<TI, TO>), grid, block, 0, ctx->stream, static_cast<const TI*>(q),      \
+  omx_launch(ctx, (sdpa_fwd_rows_kernel<TI, TO>), grid, block, 0, static_cast<const TI*>(q),      \
                      static_cast<const TI*>(k), static_cast<const TI*>(v), static_cast<TO*>(out),                 \
                      static_cast<float*>(lse), s, ctx->fault, tag)
   if (operand_dtype == OMX_F32 && out_dtype == OMX_F32) SDPA_FWD(float, float);
@@ -429,7 +429,7 @@ int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, con
       unsigned short* base = static_cast<unsigned short*>(ws);
       if (out_dtype == OMX_F32) {
         const unsigned blocks = static_cast<unsigned>(std::min<uint64_t>((n + 255) / 256, 65536));
-        hipLaunchKernelGGL(sdpa_split_output_kernel, dim3(blocks), dim3(256), 0, ctx->stream,
+        omx_launch(ctx, sdpa_split_output_kernel, dim3(blocks), dim3(256), 0,
                            static_cast<const float*>(out), base, base + n, static_cast<long>(n));
         OMX_LAUNCH_CHECK(ctx, "sdpa_split_output_kernel");
         out16 = base;
@@ -467,7 +467,7 @@ int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, con
   // The row term reads out and grad_output as they are stored; the two passes read grad_output in
   // the operands' storage type.
 #define SDPA_DELTA(TOUT, TGY)                                                                                 \
-  hipLaunchKernelGGL((sdpa_delta_kernel<TOUT, TGY>), grid, block, 0, ctx->stream, static_cast<const TOUT*>(out), \
+  omx_launch(ctx, (sdpa_delta_kernel<TOUT, TGY>), grid, block, 0, static_cast<const TOUT*>(out), \
                      static_cast<const TGY*>(gy), delta, rows, s.dim)
   if (out_dtype == OMX_F32 && gy_dtype == OMX_F32) SDPA_DELTA(float, float);
   else if (out_dtype == OMX_F32) SDPA_DELTA(float, unsigned short);
@@ -485,10 +485,10 @@ int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, con
   }
 #define SDPA_BWD(TI, TO)                                                                                              \
   do {                                                                                                                \
-    hipLaunchKernelGGL((sdpa_bwd_dq_rows_kernel<TI, TO>), grid, block, 0, ctx->stream, static_cast<const TI*>(q),     \
+    omx_launch(ctx, (sdpa_bwd_dq_rows_kernel<TI, TO>), grid, block, 0, static_cast<const TI*>(q),     \
                        static_cast<const TI*>(k), static_cast<const TI*>(v), lsef, delta, static_cast<const TI*>(gy), \
                        static_cast<TO*>(gq), s, ctx->fault, tag);                                                     \
-    hipLaunchKernelGGL((sdpa_bwd_dkv_rows_kernel<TI, TO>), kv_grid, block, 0, ctx->stream,                            \
+    omx_launch(ctx, (sdpa_bwd_dkv_rows_kernel<TI, TO>), kv_grid, block, 0,                            \
                        static_cast<const TI*>(q), static_cast<const TI*>(k), static_cast<const TI*>(v), lsef, delta,  \
                        static_cast<const TI*>(gy), static_cast<TO*>(gk), static_cast<TO*>(gv), s, ctx->fault, tag);   \
   } while (0)

@@ -564,11 +564,11 @@ int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) 
   const long bq = narrow ? 16 : 64;
   dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
   if (narrow) {
-    if (bf16_cache) hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 4, unsigned short>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
-    else hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 4, float>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, unsigned short>), grid, dim3(AT_THREADS), 0, a);
+    else omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, float>), grid, dim3(AT_THREADS), 0, a);
   } else {
-    if (bf16_cache) hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 1, unsigned short>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
-    else hipLaunchKernelGGL((sdpa32_fwd_kernel<D, 1, float>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, unsigned short>), grid, dim3(AT_THREADS), 0, a);
+    else omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, float>), grid, dim3(AT_THREADS), 0, a);
   }
   OMX_LAUNCH_CHECK(ctx, "sdpa32_fwd_kernel");
   return OMX_OK;
@@ -581,8 +581,8 @@ int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
     const bool narrow = at_narrow(ctx, planes, rows);
     const long bq = narrow ? 16 : 64;
     dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
-    if (narrow) hipLaunchKernelGGL((sdpa32_dq_kernel<D, 4>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
-    else hipLaunchKernelGGL((sdpa32_dq_kernel<D, 1>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+    if (narrow) omx_launch(ctx, (sdpa32_dq_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
+    else omx_launch(ctx, (sdpa32_dq_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);
     OMX_LAUNCH_CHECK(ctx, "sdpa32_dq_kernel");
   }
   const bool narrow = at_narrow(ctx, planes, a.tk);
@@ -601,12 +601,11 @@ int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
     a.parts = static_cast<float*>(ws);
   }
   dim3 grid(static_cast<unsigned>(blocks), planes, static_cast<unsigned>(parts));
-  if (narrow) hipLaunchKernelGGL((sdpa32_dkv_kernel<D, 4>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
-  else hipLaunchKernelGGL((sdpa32_dkv_kernel<D, 1>), grid, dim3(AT_THREADS), 0, ctx->stream, a);
+  if (narrow) omx_launch(ctx, (sdpa32_dkv_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
+  else omx_launch(ctx, (sdpa32_dkv_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);
   OMX_LAUNCH_CHECK(ctx, "sdpa32_dkv_kernel");
   if (parts > 1) {
-    hipLaunchKernelGGL(sdpa32_parts_kernel, dim3(static_cast<unsigned>((total / 4 + AT_THREADS - 1) / AT_THREADS), 2), dim3(AT_THREADS), 0,
-                       ctx->stream, a, static_cast<int>(parts), D, total);
+    omx_launch(ctx, sdpa32_parts_kernel, dim3(static_cast<unsigned>((total / 4 + AT_THREADS - 1) / AT_THREADS), 2), dim3(AT_THREADS), 0, a, static_cast<int>(parts), D, total);
     OMX_LAUNCH_CHECK(ctx, "sdpa32_parts_kernel");
   }
   return OMX_OK;

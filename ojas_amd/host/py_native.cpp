@@ -398,6 +398,282 @@ enum EntryId {
 Symbol g_symbols[] = {OMX_ENTRIES(X)};
 #undef X
 
+// ---- the backend's methods that a decoding loop calls for every token ----
+// `MiBackend` derives from a type with these methods. Each takes the well-formed call from Python's arguments to the
+// library's entry point; anything else (an operand that is no device tensor, a shape or dtype that does not fit, an
+// unknown keyword) goes to the Python method of the same name behind `_checked_`, which says what is wrong. With the
+// checks in Python a call of a 3 us launch spent 2 us on them: one token through 12 layers, 150 calls, 731 us; with
+// these methods 551 us of host time, and the device is what bounds it.
+struct Held {  // a new reference, dropped at the end of the scope
+  PyObject* o;
+  ~Held() { Py_XDECREF(o); }
+};
+
+PyObject* new_reference(PyObject* o) {
+  Py_INCREF(o);
+  return o;
+}
+
+// Positional and keyword arguments into `slot`, absent ones null; false where the names do not fit.
+template <size_t N>
+bool bind(PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames, const char* const (&names)[N], PyObject* (&slot)[N]) {
+  if (nargs > static_cast<Py_ssize_t>(N)) return false;
+  for (size_t i = 0; i < N; ++i) slot[i] = static_cast<Py_ssize_t>(i) < nargs ? args[i] : nullptr;
+  const Py_ssize_t words = kwnames ? PyTuple_GET_SIZE(kwnames) : 0;
+  for (Py_ssize_t w = 0; w < words; ++w) {
+    size_t i = 0;
+    while (i < N && PyUnicode_CompareWithASCIIString(PyTuple_GET_ITEM(kwnames, w), names[i]) != 0) ++i;
+    if (i == N || slot[i]) return false;
+    slot[i] = args[nargs + w];
+  }
+  return true;
+}
+
+const Tensor* tensor_in(PyObject* o) { return o && Py_TYPE(o) == &TensorType ? reinterpret_cast<const Tensor*>(o) : nullptr; }
+// A float tensor with elements, as the validators ask of every operand.
+const Tensor* floats_in(PyObject* o) {
+  const Tensor* t = tensor_in(o);
+  return t && (t->dtype == 0 || t->dtype == 1) && t->numel > 0 ? t : nullptr;
+}
+Py_ssize_t rank(const Tensor* t) { return PyTuple_GET_SIZE(t->shape); }
+Py_ssize_t axis(const Tensor* t, Py_ssize_t i) { return PyLong_AsSsize_t(PyTuple_GET_ITEM(t->shape, i)); }
+Py_ssize_t last_axis(const Tensor* t) { return axis(t, rank(t) - 1); }
+// An optional dtype (None and absent: `otherwise`), -1 where it is none.
+int dtype_in(PyObject* o, int otherwise) {
+  if (!o || o == Py_None) return otherwise;
+  if (!PyLong_CheckExact(o)) return -1;
+  const long v = PyLong_AsLong(o);
+  if (v == -1 && PyErr_Occurred()) PyErr_Clear();
+  return v >= 0 && v <= 3 ? static_cast<int>(v) : -1;
+}
+// A whole number from 0 to 2^62, -1 where it is none.
+long long count_in(PyObject* o) {
+  if (!o || !PyLong_CheckExact(o)) return -1;
+  const long long v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) PyErr_Clear();
+  return v >= 0 && v <= (1ll << 62) ? v : -1;
+}
+
+PyObject* new_tensor(PyObject* backend, Context* c, PyObject* shape /* stolen */, int dtype) {
+  if (!shape) return nullptr;
+  const Py_ssize_t n = elements(shape);
+  void* p = nullptr;
+  const int32_t rc = c->ctx ? p_alloc(c->ctx, static_cast<uint64_t>(n > 1 ? n : 1) * kSizes[dtype], &p) : OMX_BACKEND;
+  if (rc != OMX_OK) {
+    Py_DECREF(shape);
+    return raise(c->ctx, rc);
+  }
+  Tensor* t = make_tensor(backend, c, reinterpret_cast<unsigned long long>(p), shape, n, dtype, true);
+  if (!t) p_free(c->ctx, p);
+  return reinterpret_cast<PyObject*>(t);
+}
+// x's shape with its last axis (or, with `append`, one more axis) of `n`.
+PyObject* shape_with(const Tensor* x, Py_ssize_t n, bool append) {
+  const Py_ssize_t lead = rank(x) - (append ? 0 : 1);
+  PyObject* shape = PyTuple_New(lead + 1);
+  if (!shape) return nullptr;
+  for (Py_ssize_t i = 0; i < lead; ++i) {
+    PyObject* a = PyTuple_GET_ITEM(x->shape, i);
+    Py_INCREF(a);
+    PyTuple_SET_ITEM(shape, i, a);
+  }
+  PyObject* a = PyLong_FromSsize_t(n);
+  if (!a) {
+    Py_DECREF(shape);
+    return nullptr;
+  }
+  PyTuple_SET_ITEM(shape, lead, a);
+  return shape;
+}
+PyObject* shape_of(const Tensor* x) {
+  Py_INCREF(x->shape);
+  return x->shape;
+}
+template <typename T = void>
+T* memory(const Tensor* t) {
+  return reinterpret_cast<T*>(t->ptr);
+}
+template <typename T = void>
+T* memory(const Held& h) {
+  return reinterpret_cast<T*>(reinterpret_cast<const Tensor*>(h.o)->ptr);
+}
+
+// The call's context (a reference) and, where the fast path does not apply, its Python method.
+Context* context_of(PyObject* self) {
+  static PyObject* name = PyUnicode_InternFromString("_context");
+  PyObject* c = PyObject_GetAttr(self, name);
+  if (c && Py_TYPE(c) != &ContextType) Py_CLEAR(c);
+  if (!c) PyErr_Clear();
+  return reinterpret_cast<Context*>(c);
+}
+PyObject* in_python(PyObject* self, PyObject* name, PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames) {
+  Held method{PyObject_GetAttr(self, name)};
+  return method.o ? PyObject_Vectorcall(method.o, args, nargs, kwnames) : nullptr;
+}
+// The library call without the interpreter lock; null with the error set where it refuses.
+template <typename F>
+bool without_lock(Context* c, F&& call) {
+  int32_t rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = call(c->ctx);
+  Py_END_ALLOW_THREADS
+  if (rc != OMX_OK) raise(c->ctx, rc);
+  return rc == OMX_OK;
+}
+
+#define OMX_METHOD(name) PyObject* m_##name(PyObject* self, PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames)
+#define OMX_IN_PYTHON(name)                                                 \
+  do {                                                                      \
+    static PyObject* checked = PyUnicode_InternFromString("_checked_" #name); \
+    return in_python(self, checked, args, nargs, kwnames);                  \
+  } while (0)
+#define OMX_CALL(name) (reinterpret_cast<decltype(&::name)>(*g_symbols[ID_##name].address))
+
+OMX_METHOD(linear_forward) {
+  static const char* const names[] = {"x", "w", "out_dtype"};
+  PyObject* slot[3];
+  const bool bound = bind(args, nargs, kwnames, names, slot);
+  const Tensor *x = bound ? floats_in(slot[0]) : nullptr, *w = bound ? floats_in(slot[1]) : nullptr;
+  const int dtype = bound ? dtype_in(slot[2], 0) : -1;
+  Held ctx{x && w ? reinterpret_cast<PyObject*>(context_of(self)) : nullptr};
+  if (!ctx.o || dtype < 0 || rank(x) < 1 || rank(w) != 2 || last_axis(x) != axis(w, 1)) OMX_IN_PYTHON(linear_forward);
+  Context* c = reinterpret_cast<Context*>(ctx.o);
+  const Py_ssize_t kin = axis(w, 1), nout = axis(w, 0);
+  Held y{new_tensor(self, c, shape_with(x, nout, false), dtype)};
+  if (!y.o || !without_lock(c, [&](omx_ctx* o) {
+        return OMX_CALL(omx_linear_forward)(o, memory(x), x->dtype, memory(w), w->dtype, memory(y), dtype, x->numel / kin, kin, nout);
+      }))
+    return nullptr;
+  return new_reference(y.o);
+}
+
+OMX_METHOD(linear_gelu_forward) {
+  static const char* const names[] = {"x", "w", "tanh_form"};
+  PyObject* slot[3];
+  const bool bound = bind(args, nargs, kwnames, names, slot);
+  const Tensor *x = bound ? floats_in(slot[0]) : nullptr, *w = bound ? floats_in(slot[1]) : nullptr;
+  Held ctx{x && w ? reinterpret_cast<PyObject*>(context_of(self)) : nullptr};
+  if (!ctx.o || rank(x) < 1 || rank(w) != 2 || last_axis(x) != axis(w, 1) || (slot[2] && !PyBool_Check(slot[2])))
+    OMX_IN_PYTHON(linear_gelu_forward);
+  Context* c = reinterpret_cast<Context*>(ctx.o);
+  const Py_ssize_t kin = axis(w, 1), nout = axis(w, 0);
+  Held u{new_tensor(self, c, shape_with(x, nout, false), 1)};
+  Held act{u.o ? new_tensor(self, c, shape_with(x, nout, false), 1) : nullptr};
+  if (!act.o || !without_lock(c, [&](omx_ctx* o) {
+        return OMX_CALL(omx_linear_gelu_forward)(o, memory(x), memory(w), x->dtype, memory(u), memory(act), x->numel / kin, kin, nout,
+                                                 slot[2] == Py_True);
+      }))
+    return nullptr;
+  return PyTuple_Pack(2, u.o, act.o);
+}
+
+OMX_METHOD(residual_add_rms_norm_forward) {
+  static const char* const names[] = {"x", "y", "w", "eps", "out_dtype"};
+  PyObject* slot[5];
+  const bool bound = bind(args, nargs, kwnames, names, slot);
+  const Tensor *x = bound ? floats_in(slot[0]) : nullptr, *y = bound ? floats_in(slot[1]) : nullptr;
+  const Tensor* w = bound ? floats_in(slot[2]) : nullptr;
+  const int dtype = y ? dtype_in(slot[4], y->dtype) : -1;
+  Held ctx{x && y && w ? reinterpret_cast<PyObject*>(context_of(self)) : nullptr};
+  if (!ctx.o || dtype < 0 || rank(x) < 1 || (slot[3] && !PyFloat_CheckExact(slot[3]))) OMX_IN_PYTHON(residual_add_rms_norm_forward);
+  Context* c = reinterpret_cast<Context*>(ctx.o);
+  const Py_ssize_t dim = last_axis(x);
+  const float eps = slot[3] ? static_cast<float>(PyFloat_AS_DOUBLE(slot[3])) : 1e-6f;
+  Held total{new_tensor(self, c, shape_of(x), 0)};
+  Held normed{total.o ? new_tensor(self, c, shape_of(x), dtype) : nullptr};
+  if (!normed.o || !without_lock(c, [&](omx_ctx* o) {
+        return OMX_CALL(omx_residual_add_rms_norm_forward)(o, memory(x), x->dtype, memory(y), y->dtype, memory<float>(w), memory<float>(total),
+                                                           memory(normed), dtype, x->numel / dim, dim, eps);
+      }))
+    return nullptr;
+  return PyTuple_Pack(2, total.o, normed.o);
+}
+
+OMX_METHOD(to_bf16) {
+  static const char* const names[] = {"x"};
+  PyObject* slot[1];
+  const Tensor* x = bind(args, nargs, kwnames, names, slot) ? floats_in(slot[0]) : nullptr;
+  Held ctx{x ? reinterpret_cast<PyObject*>(context_of(self)) : nullptr};
+  if (!ctx.o) OMX_IN_PYTHON(to_bf16);
+  Context* c = reinterpret_cast<Context*>(ctx.o);
+  Held y{new_tensor(self, c, shape_of(x), 1)};
+  if (!y.o || !without_lock(c, [&](omx_ctx* o) { return OMX_CALL(omx_to_bf16)(o, memory<float>(x), memory(y), x->numel); })) return nullptr;
+  return new_reference(y.o);
+}
+
+OMX_METHOD(embedding_forward) {
+  static const char* const names[] = {"table", "ids", "out_dtype"};
+  PyObject* slot[3];
+  const bool bound = bind(args, nargs, kwnames, names, slot);
+  const Tensor *table = bound ? floats_in(slot[0]) : nullptr, *ids = bound ? tensor_in(slot[1]) : nullptr;
+  const int dtype = bound ? dtype_in(slot[2], 0) : -1;
+  Held ctx{table && ids ? reinterpret_cast<PyObject*>(context_of(self)) : nullptr};
+  if (!ctx.o || dtype < 0 || rank(table) != 2 || ids->dtype != 2 || ids->numel < 1) OMX_IN_PYTHON(embedding_forward);
+  Context* c = reinterpret_cast<Context*>(ctx.o);
+  const Py_ssize_t vocab = axis(table, 0), dim = axis(table, 1);
+  Held y{new_tensor(self, c, shape_with(ids, dim, true), dtype)};
+  if (!y.o || !without_lock(c, [&](omx_ctx* o) {
+        return OMX_CALL(omx_embedding_forward)(o, memory(table), table->dtype, memory(ids), memory(y), dtype, ids->numel, vocab, dim);
+      }))
+    return nullptr;
+  return new_reference(y.o);
+}
+
+OMX_METHOD(kv_cache_write) {
+  static const char* const names[] = {"cache", "src", "at"};
+  PyObject* slot[3];
+  const bool bound = bind(args, nargs, kwnames, names, slot);
+  const Tensor *cache = bound ? floats_in(slot[0]) : nullptr, *src = bound ? floats_in(slot[1]) : nullptr;
+  const long long at = bound ? count_in(slot[2]) : -1;
+  Held ctx{cache && src ? reinterpret_cast<PyObject*>(context_of(self)) : nullptr};
+  if (!ctx.o || at < 0 || rank(cache) != 4 || rank(src) != 4 || src->dtype != 0 || axis(src, 0) != axis(cache, 0) ||
+      axis(src, 2) != axis(cache, 2) || axis(src, 3) != axis(cache, 3) || axis(src, 1) > axis(cache, 1))
+    OMX_IN_PYTHON(kv_cache_write);
+  Context* c = reinterpret_cast<Context*>(ctx.o);
+  if (!without_lock(c, [&](omx_ctx* o) {
+        return OMX_CALL(omx_kv_cache_write)(o, memory(cache), cache->dtype, memory<float>(src), axis(cache, 0), axis(cache, 1), axis(cache, 2),
+                                            axis(cache, 3), axis(src, 1), at);
+      }))
+    return nullptr;
+  Py_RETURN_NONE;
+}
+
+OMX_METHOD(cached_attention_forward) {
+  static const char* const names[] = {"q", "k_cache", "v_cache", "kv_len", "window"};
+  PyObject* slot[5];
+  const bool bound = bind(args, nargs, kwnames, names, slot);
+  const Tensor *q = bound ? floats_in(slot[0]) : nullptr, *k = bound ? floats_in(slot[1]) : nullptr;
+  const Tensor* v = bound ? floats_in(slot[2]) : nullptr;
+  const long long kv_len = bound ? count_in(slot[3]) : -1;
+  const long long window = bound && slot[4] && slot[4] != Py_None ? count_in(slot[4]) : 0;
+  Held ctx{q && k && v ? reinterpret_cast<PyObject*>(context_of(self)) : nullptr};
+  if (!ctx.o || kv_len < 0 || window < 0 || (slot[4] && slot[4] != Py_None && window == 0) || rank(q) != 4 || rank(k) != 4 ||
+      rank(v) != 4 || q->dtype != 0 || k->dtype != v->dtype)
+    OMX_IN_PYTHON(cached_attention_forward);
+  const Py_ssize_t b = axis(q, 0), tq = axis(q, 1), h = axis(q, 2), d = axis(q, 3), cap = axis(k, 1), hkv = axis(k, 2);
+  const long long span = window && window < kv_len && tq + window - 1 < kv_len ? tq + window - 1 : kv_len;
+  bool fits = axis(k, 0) == b && axis(k, 3) == d && h % hkv == 0 && kv_len >= tq && span <= cap;
+  for (Py_ssize_t i = 0; i < 4; ++i) fits &= axis(k, i) == axis(v, i);
+  if (!fits) OMX_IN_PYTHON(cached_attention_forward);
+  Context* c = reinterpret_cast<Context*>(ctx.o);
+  Held out{new_tensor(self, c, shape_of(q), 0)};
+  if (!out.o || !without_lock(c, [&](omx_ctx* o) {
+        return OMX_CALL(omx_cached_attention_forward)(o, memory<float>(q), memory(k), memory(v), k->dtype, memory<float>(out), b, tq, h, hkv, d,
+                                                      cap, kv_len, window);
+      }))
+    return nullptr;
+  return new_reference(out.o);
+}
+
+#define OMX_METHODS(X)                                                                                              \
+  X(linear_forward) X(linear_gelu_forward) X(residual_add_rms_norm_forward) X(to_bf16) X(embedding_forward)        \
+  X(kv_cache_write) X(cached_attention_forward)
+#define X(name) \
+  {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&m_##name)), METH_FASTCALL | METH_KEYWORDS, "See `_checked_" #name "`."},
+PyMethodDef backend_methods[] = {OMX_METHODS(X){nullptr, nullptr, 0, nullptr}};
+#undef X
+PyTypeObject MethodsType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
 // load(path, error_type): opens the library and finds every entry point.
 PyObject* load(PyObject*, PyObject* args) {
   const char* path;
@@ -455,12 +731,20 @@ PyMODINIT_FUNC PyInit__native(void) {
   TensorType.tp_methods = tensor_methods;
   TensorType.tp_members = tensor_members;
   TensorType.tp_getset = tensor_getset;
-  if (PyType_Ready(&ContextType) < 0 || PyType_Ready(&TensorType) < 0) return nullptr;
+  MethodsType.tp_name = "ojas_amd._native.Methods";
+  MethodsType.tp_doc = "The native methods of the backend class that derives from it.";
+  MethodsType.tp_basicsize = sizeof(PyObject);
+  MethodsType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+  MethodsType.tp_new = PyType_GenericNew;
+  MethodsType.tp_methods = backend_methods;
+  if (PyType_Ready(&ContextType) < 0 || PyType_Ready(&TensorType) < 0 || PyType_Ready(&MethodsType) < 0) return nullptr;
   PyObject* m = PyModule_Create(&module);
   if (!m) return nullptr;
   Py_INCREF(&ContextType);
   Py_INCREF(&TensorType);
-  if (PyModule_AddObject(m, "Context", reinterpret_cast<PyObject*>(&ContextType)) < 0 ||
+  Py_INCREF(&MethodsType);
+  if (PyModule_AddObject(m, "Methods", reinterpret_cast<PyObject*>(&MethodsType)) < 0 ||
+      PyModule_AddObject(m, "Context", reinterpret_cast<PyObject*>(&ContextType)) < 0 ||
       PyModule_AddObject(m, "DeviceTensor", reinterpret_cast<PyObject*>(&TensorType)) < 0)
     return nullptr;
   return m;

@@ -23,3 +23,32 @@ def test_refusals(monkeypatch):
         _native.omx_sync(5)  # not a context
     with pytest.raises(TypeError):
         _native.omx_sync(_native.Context(0), np.zeros(3))  # argument count
+
+
+def test_native_methods_leave_what_does_not_fit_to_the_python_ones():
+    """A call that is not well-formed reaches the checks of the Python method, whatever is wrong with it."""
+    from ojas_amd.backend import DTYPE, PLACEMENT, U32, MiBackend
+
+    be = MiBackend.__new__(MiBackend)  # no device: nothing here gets as far as the library
+    be._ctx, be._context = None, _native.Context(0)
+
+    def dev(*shape, dtype=BF16):
+        return DeviceTensor(be, 4096, shape, dtype, owns=False)
+
+    host = np.zeros((2, 3), np.float32)
+    for code, call in [
+        (SHAPE, lambda: be.linear_forward(dev(2, 3), dev(4, 5))), (SHAPE, lambda: be.linear_forward(dev(2, 3), dev(3))),
+        (SHAPE, lambda: be.linear_forward(dev(0, 3), dev(4, 3))), (DTYPE, lambda: be.linear_forward(dev(2, 3, dtype=U32), dev(4, 3))),
+        (PLACEMENT, lambda: be.linear_forward(host, host)), (SHAPE, lambda: be.embedding_forward(dev(4), dev(2, dtype=U32))),
+        (DTYPE, lambda: be.embedding_forward(dev(4, 3), dev(2))), (SHAPE, lambda: be.kv_cache_write(dev(1, 4, 2, 8), dev(1, 1, 2, 4, dtype=F32), 0)),
+        (DTYPE, lambda: be.kv_cache_write(dev(1, 4, 2, 8), dev(1, 1, 2, 8), 0)),
+        (SHAPE, lambda: be.cached_attention_forward(dev(1, 1, 4, 8, dtype=F32), dev(1, 4, 3, 8), dev(1, 4, 3, 8), 1)),
+        (SHAPE, lambda: be.cached_attention_forward(dev(1, 1, 4, 8, dtype=F32), dev(1, 4, 2, 8), dev(1, 4, 2, 8), 1, window=0)),
+        (DTYPE, lambda: be.cached_attention_forward(dev(1, 1, 4, 8), dev(1, 4, 2, 8), dev(1, 4, 2, 8), 1))]:
+        with pytest.raises(OjasError) as e:
+            call()
+        assert e.value.code == code
+    for call in (lambda: be.linear_forward(dev(2, 3), dev(4, 3), nonsense=1), lambda: be.linear_forward(dev(2, 3)),
+                 lambda: be.linear_forward(dev(2, 3), dev(4, 3), None, 1), lambda: be.linear_forward(dev(2, 3), dev(4, 3), x=1)):
+        with pytest.raises(TypeError):
+            call()
