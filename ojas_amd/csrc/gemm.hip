@@ -399,6 +399,46 @@ int32_t launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km) {
   return OMX_OK;
 }
 
+// How often a bf16 product of `tiles` tiles over `ksteps` steps of 64 columns is split over K on the 256 x 128 and
+// 128 x 128 direct-to-LDS tiles: two workgroups per compute unit, eight steps or more each, a power of two (a split
+// then stays on one XCD, see gemm_dma_kernel).
+int dma_splits(long tiles, int ksteps) {
+  int splits = static_cast<int>((512 + tiles - 1) / tiles);
+  if (splits > ksteps / 8) splits = ksteps / 8;
+  if (splits < 1) splits = 1;
+  int p2 = 1;
+  while (p2 * 2 <= splits + splits / 4) p2 *= 2;  // 7..9 -> 8, 10..12 -> 8, 13..16 -> 16
+  return p2;
+}
+
+// What a product takes on one of the direct-to-LDS tilings below 256 x 256, in us: rounds of tiles over the chip, each
+// K steps long, and a split's second launch with its partial sums (8 bytes per output element and split, out of the
+// caches). The smaller tiles' rounds count whole (the last one's latency is not hidden), the others' in part (two or
+// three workgroups share a compute unit). Fitted to 512 .. 8192 rows, 512 .. 3072 columns over K = 512 .. 16384 in
+// all three layouts, within 15 % nearly everywhere.
+double dma_us(int variant, long m, long n, long batches, int ksteps, int splits, bool a_km, bool activation, long cus) {
+  int bm, bn;
+  omx_gemm_dma_tile(variant, &bm, &bn);
+  const long groups = ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batches * splits;
+  const double rounds = variant >= 7 || groups < cus ? static_cast<double>((groups + cus - 1) / cus)
+                                                     : static_cast<double>(groups) / static_cast<double>(cus);
+  // (a larger tile's store pass takes longer, an activation's more so; 64 columns of a k-major row are one cache line)
+  const double base = variant == 8 ? 3.0 : variant == 7 ? 3.5 : variant == 6 ? (activation ? 5.0 : 4.0) : activation ? 7.5 : 4.5;
+  const double step = variant == 8 ? (a_km ? 0.23 : 0.19) : variant == 7 ? 0.31 : variant == 6 ? 0.65 : 0.95;
+  return base + step * rounds * ((ksteps + splits - 1) / splits) +
+         (splits > 1 ? 6.0 + 1e-6 * static_cast<double>(m * n * splits) : 0.0);
+}
+
+// The cheapest split of a product over tiling 6, 7 or 8, at most `limit` ways.
+int small_tile_splits(int variant, long m, long n, long batches, int ksteps, int limit, bool a_km, bool activation, long cus) {
+  int best = 1;
+  for (int s = 2; s <= limit && ksteps / s >= 8; s *= 2)
+    if (dma_us(variant, m, n, batches, ksteps, s, a_km, activation, cus) <
+        dma_us(variant, m, n, batches, ksteps, best, a_km, activation, cus))
+      best = s;
+  return best;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
@@ -475,14 +515,15 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   const bool thin = operand_dtype == OMX_BF16 && ctx->gemm_thin && !(epi && epi->mode != OMX_EPI_NONE) &&
                     omx_gemm_thin_eligible(g, a_km, b_km);
   // Few rows (a decoder's linear layers): K shared between a workgroup's waves, no tile of 128 rows.
-  const bool skinny = operand_dtype == OMX_BF16 && !thin && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0 &&
-                      omx_gemm_skinny_eligible(ctx, g, a_km, b_km);
+  const double skinny_us = operand_dtype == OMX_BF16 && !thin && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
+                               ? omx_gemm_skinny_us(ctx, g, a_km, b_km) : -1.0;
+  bool skinny = skinny_us >= 0.0;
   // f32 outputs of less than a few rounds of 128 x 128 tiles.
   int frag32 = -1;
   if (operand_dtype == OMX_F32 && ctx->gemm_dma_mode == 1 && !(epi && epi->mode != OMX_EPI_NONE))
     frag32 = omx_gemm_frag32_tile(ctx, g, a_km, b_km);
-  int dma_variant = -1;
-  if (!thin && !skinny && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) {
+  int dma_variant = -1, small_splits = 0;
+  if (!thin && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) {
     const int mode = ctx->gemm_dma_mode;
     if (mode == 1 && ctx->gemm_forced_tiling >= 0) {
       dma_variant = ctx->gemm_forced_tiling;
@@ -559,9 +600,46 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       } else {
         dma_variant = 3;
       }
+      // A few hundred to a few thousand tokens, or a model some hundred wide, make less than a round or two of those
+      // tiles. Two smaller ones in 64-column steps (whole cache lines of a k-contiguous row, three stages), where
+      // they take a tenth less than the choice above, or a fifth less than the few-row kernel, whose
+      // workgroups have all of cold weights in flight at once:
+      //   7  128 x 64, four waves, two workgroups per compute unit;
+      //   8  64 x 64, four waves, three per compute unit.
+      // A K step costs them 1.5 to 2 times the LDS traffic per product, so full rounds of the larger tiles stay there.
+      // 3500 x 512 over K = 512 / 2048: 10.0 / 27.6 -> 5.8 / 14.4 us; 1024 x 3072 over 768 with GELU 17.3 -> 11.7;
+      // 1024 x 768 over 768: 9.1 -> 5.1; six weight gradients of 512 x 512 over 3500: 54 -> 25. Scratch for a split
+      // stays within what the choice above would have taken.
+      if (dma_variant < 9) {
+        const int ks = static_cast<int>(ksteps64);
+        int bm = 128, bn = 128;
+        if (dma_variant >= 0) omx_gemm_dma_tile(dma_variant, &bm, &bn);
+        const long tiles = ((g.M + bm - 1l) / bm) * ((g.N + bn - 1l) / bn);
+        const bool may_split = plain && !skinny && unbatched && tiles < 256 && ks >= 32;
+        const int before = may_split && dma_variant >= 0 ? dma_splits(tiles, ks) : 1;
+        const int limit = may_split && dma_variant < 0 ? static_cast<int>(std::min<long>((512 + tiles - 1) / tiles, ks / 8))
+                                                       : before;
+        double best = skinny            ? 0.8 * skinny_us
+                      : dma_variant < 0 ? 1e30
+                                        : 0.9 * dma_us(dma_variant, g.M, g.N, g.batches, ks, before, a_km, !plain, cus);
+        for (int v = 6; v <= 8; ++v) {
+          if (v == dma_variant) continue;
+          const int s = small_tile_splits(v, g.M, g.N, g.batches, ks, limit, a_km, !plain, cus);
+          const double us = dma_us(v, g.M, g.N, g.batches, ks, s, a_km, !plain, cus);
+          if (us < best) {
+            best = us;
+            dma_variant = v;
+            small_splits = s;
+            skinny = false;
+          }
+        }
+      }
+      if (skinny) dma_variant = -1;
     }
     else if (mode == 3) dma_variant = 3;
     else if (mode == 4) dma_variant = 6;
+    else if (mode == 7) dma_variant = 7;
+    else if (mode == 8) dma_variant = 8;
     else if (mode == 9) dma_variant = 9;
     else if (mode == 10) dma_variant = 10;
     if (dma_variant >= 9 && !omx_gemm_w4_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) dma_variant = 3;
@@ -622,10 +700,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       splits = static_cast<int>(((g.batches == 1 ? 512 : 1024) + all_tiles - 1) / all_tiles);
       if (splits > ksteps / min_steps) splits = ksteps / min_steps;
       if (splits < 1) splits = 1;
-      if (dma_variant >= 0) {  // a power of two, so that a split stays on one XCD (see gemm_dma_kernel)
-        int p2 = 1;
-        while (p2 * 2 <= splits + splits / 4) p2 *= 2;  // 7..9 -> 8, 10..12 -> 8, 13..16 -> 16
-        splits = p2;
+      if (dma_variant >= 0) {
+        splits = dma_splits(all_tiles, ksteps);
         if (dma_variant >= 9) {
           // One workgroup per compute unit: what counts is how full the last round of workgroups is
           // (192 tiles split in two are 384 workgroups on 256 units, a round and a half; split in
@@ -647,6 +723,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
         }
       }
     }
+    if (small_splits > 0) splits = small_splits;  // chosen with the tiling
+    else if (dma_variant == 7 || dma_variant == 8) splits = 1;
     g.ksteps_per_split = (ksteps + splits - 1) / splits;
     if (dma_variant >= 9) g.ksteps_per_split += g.ksteps_per_split & 1;  // its K loop takes steps in pairs
     g.splits = (ksteps + g.ksteps_per_split - 1) / g.ksteps_per_split;
@@ -769,8 +847,8 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value) {
     return OMX_OK;
   }
   if (name && strcmp(name, "gemm_dma") == 0) {
-    if (value != 0 && value != 1 && value != 3 && value != 4 && value != 9 && value != 10)
-      return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: gemm_dma takes 0, 1, 3, 4, 9 or 10");
+    if (value != 0 && value != 1 && value != 3 && value != 4 && value != 7 && value != 8 && value != 9 && value != 10)
+      return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: gemm_dma takes 0, 1, 3, 4, 7, 8, 9 or 10");
     ctx->gemm_dma_mode = static_cast<int>(value);
     return OMX_OK;
   }

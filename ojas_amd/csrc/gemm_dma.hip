@@ -57,8 +57,8 @@ bool omx_gemm_w4_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain) {
 }
 
 void omx_gemm_dma_tile(int variant, int* bm, int* bn) {
-  *bm = variant == 6 ? 128 : 256;
-  *bn = variant == 9 ? 256 : variant == 10 ? 192 : 128;
+  *bm = variant == 6 || variant == 7 ? 128 : variant == 8 ? 64 : 256;
+  *bn = variant == 9 ? 256 : variant == 10 ? 192 : variant == 7 || variant == 8 ? 64 : 128;
 }
 
 

@@ -193,7 +193,7 @@ gemm_dma_kernel(GemmArgs g) {
     constexpr int PPR = TN * 8;  // 4-column pieces per row
     // A block that lies wholly inside the output takes a straight-line store loop (compiled for
     // the two forms the dispatcher picks by itself); edge blocks and the other forms go piece by piece.
-    constexpr bool kFastStores = (DBK == 32 && TM * TN <= 4) || NW == 6;
+    constexpr bool kFastStores = TM * TN <= 4;
     const int grow0 = m0 + (wm * TM + tm) * 32, gcol0 = n0 + wn * TN * 32;
     bool stored = false;
     if constexpr (kFastStores) {
@@ -272,6 +272,8 @@ int32_t launch_variant(omx_ctx* ctx, const GemmArgs& g, int variant) {
     return omx_fail(ctx, OMX_SHAPE, "gemm: no one-wave-per-SIMD kernel for this operand layout");
   }
   if (variant == 6) return launch_dma<A_KM, B_KM, 2, 2, 2, 2, 32, 3>(ctx, g);
+  if (variant == 7) return launch_dma<A_KM, B_KM, 2, 2, 2, 1, 64, 3>(ctx, g);
+  if (variant == 8) return launch_dma<A_KM, B_KM, 2, 2, 1, 1, 64, 3>(ctx, g);
   return launch_dma<A_KM, B_KM, 4, 2, 2, 2, 32, 3>(ctx, g);
 }
 

@@ -147,9 +147,11 @@ int32_t launch_skinny(omx_ctx* ctx, const GemmArgs& g) {
 
 }  // namespace
 
-bool omx_gemm_skinny_eligible(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km) {
-  if (a_km || b_km || g.K % 32 != 0 || !g.a_vec || !g.b_vec) return false;
-  return skinny_tile(g, ctx->cu_count > 0 ? ctx->cu_count : 256) >= 0;
+// What the product takes here, in us (see skinny_tile); negative: not one for this kernel.
+double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km) {
+  if (a_km || b_km || g.K % 32 != 0 || !g.a_vec || !g.b_vec) return -1.0;
+  const int t = skinny_tile(g, ctx->cu_count > 0 ? ctx->cu_count : 256);
+  return t < 0 ? -1.0 : 2.5 + 1e-3 * g.K * (SKINNY_TILES[t].mb + SKINNY_TILES[t].nb);
 }
 
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g) {

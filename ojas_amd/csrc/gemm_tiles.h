@@ -94,6 +94,13 @@ struct StepBase<true, true> {
   }
 };
 
+// What K row kr of a k-major tile XORs its 16-byte slots with: the four rows of a transposing read 64 bytes apart in the
+// 256 bytes that the banks span. (A row of 64 elements is half of that, so rows 0 and 2, 1 and 3 have to part.)
+template <int ROWS>
+__device__ __forceinline__ int km_swizzle(int kr) {
+  return ROWS == 64 ? (kr >> 1 & 1) * 4 : (kr & 3) * 4;
+}
+
 // One operand's loads: ROWS x BK bf16 per step, one wave instruction per KiB. Rows past the end are clamped in the
 // offset, so edge tiles take this form too (a k-major operand's last 16-byte chunk may reach past its last column into
 // the padding of the row, which is at least 16 bytes aligned; those values only meet outputs that are not stored).
@@ -124,7 +131,7 @@ struct TileLoadsOff {
         constexpr int CPR = ROWS / 8;
         const int idx = q * 64 + lane;
         const int kr = idx / CPR, slot = idx % CPR;
-        const int mc = slot ^ ((kr & 3) * 4);
+        const int mc = slot ^ km_swizzle<ROWS>(kr);
         int gm = mc * 8;
         gm = row0 + gm < rows ? gm : 0;
         off[i] = static_cast<unsigned>(kr) * static_cast<unsigned>(ld * 2) + gm * 2;
@@ -154,7 +161,7 @@ __device__ __forceinline__ int frag_offset(int row_base, int kk, int lane) {
     const int s = lane & 15, half = (lane >> 4) & 1, g = lane >> 5;
     const int kr = kk * 16 + g * 8 + (s >> 2);
     const int col = row_base + half * 16 + (s & 3) * 4;
-    const int slot = (col >> 3) ^ (((s >> 2) & 3) * 4);
+    const int slot = (col >> 3) ^ km_swizzle<ROWS>(kr);
     return kr * (ROWS * 2) + slot * 16 + (col & 7) * 2;
   }
 }

@@ -260,6 +260,68 @@ def test_reductions_of_any_length_end_inside_a_step(be, mode, tokens, m, n, pitc
     assert float(np.max(np.abs(got - want))) <= 2e-5 * max(1.0, float(np.max(np.abs(want))))
 
 
+@pytest.mark.parametrize("mode", [7, 8])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("m,k,n", [(64, 64, 64), (1, 128, 1), (65, 192, 63), (130, 256, 200), (333, 2048, 72)])
+def test_small_direct_to_lds_tiles(be, mode, layout, m, k, n):
+    """The 128 x 64 and 64 x 64 tiles: one tile, one row and column, a row and a column past a tile, fewer K steps than
+    stages; f32, bf16 and accumulated outputs, and a batch. Against the f64 product of the same bf16 operands: every
+    product is exact in f32, so what is left is f32 sums (1e-5 of the largest value) or one bf16 rounding (2^-8)."""
+    from ojas_amd.backend import BF16
+
+    print(f"gemm small tiles mode {mode} {layout} {m}x{k}x{n}", flush=True)
+    rng = np.random.default_rng(m * k + n)
+    lda, ldb = (m + 7) // 8 * 8, (n + 7) // 8 * 8
+    ta, tb = layout[0] == "T", layout[1] == "T"
+    a = orc.round_bf16((rng.standard_normal((2, k, lda) if ta else (2, m, k)) * 0.5).astype(np.float32).ravel()).reshape((2, k, lda) if ta else (2, m, k))
+    b = orc.round_bf16((rng.standard_normal((2, k, ldb) if tb else (2, n, k)) * 0.5).astype(np.float32).ravel()).reshape((2, k, ldb) if tb else (2, n, k))
+    fa = a.astype(np.float64)[:, :, :m].transpose(0, 2, 1) if ta else a.astype(np.float64)
+    fb = b.astype(np.float64)[:, :, :n] if tb else b.astype(np.float64).transpose(0, 2, 1)
+    want = fa @ fb
+    sa, sb = ((1, lda) if ta else (k, 1)), ((ldb, 1) if tb else (1, k))
+    c0 = rng.standard_normal((m, n)).astype(np.float32)
+    da, db, dc = be.upload(a, BF16), be.upload(b, BF16), be.upload(c0)
+    pad = (m * n + 3) // 4 * 4
+    be.set_option("gemm_dma", mode)
+    try:
+        plain = be.download(be.gemm(da, sa, db, sb, m, k, n))
+        short = be.download_f32(be.gemm(da, sa, db, sb, m, k, n, out_dtype=BF16))
+        be.gemm(da, sa, db, sb, m, k, n, c=dc)
+        both = be.download(be.gemm_strided_batch(da, sa, db, sb, m, k, n, 2, (a[0].size, b[0].size, pad)))
+    finally:
+        be.set_option("gemm_dma", 1)
+    top = max(1.0, float(np.max(np.abs(want))))
+    assert float(np.max(np.abs(plain - want[0]))) <= 1e-5 * top
+    assert float(np.max(np.abs(short - want[0]))) <= 2.0 ** -8 * top
+    assert float(np.max(np.abs(be.download(dc) - c0 - want[0]))) <= 1e-5 * top
+    for j in range(2):
+        assert float(np.max(np.abs(both[j * pad:j * pad + m * n].reshape(m, n) - want[j]))) <= 1e-5 * top
+
+
+@pytest.mark.parametrize("mode", [7, 8])
+@pytest.mark.parametrize("rows,kin,nout", [(64, 64, 64), (70, 192, 100), (300, 512, 520)])
+def test_small_direct_to_lds_tiles_with_gelu(be, mode, rows, kin, nout):
+    """The activation's store pass on the small tiles gives the bits of the 256 x 128 tiles' (one K order in both)."""
+    from ojas_amd.backend import BF16
+
+    rng = np.random.default_rng(rows)
+    x = be.upload(orc.round_bf16((rng.standard_normal(rows * kin) * 0.5).astype(np.float32)).reshape(rows, kin), BF16)
+    w = be.upload(orc.round_bf16((rng.standard_normal(nout * kin) * 0.2).astype(np.float32)).reshape(nout, kin), BF16)
+    got = {}
+    for m in (3, mode):
+        be.set_option("gemm_dma", m)
+        got[m] = [be.download(t) for t in be.linear_gelu_forward(x, w)]
+    be.set_option("gemm_dma", 1)
+    for mine, theirs in zip(got[mode], got[3]):
+        assert np.array_equal(mine, theirs)
+
+
+@pytest.mark.parametrize("mode", [7, 8])
+@pytest.mark.parametrize("tokens,m,n,pitch", [(1, 64, 64, 64), (65, 72, 64, 72), (127, 57, 192, 64), (3500, 512, 512, 512)])
+def test_small_tiles_end_a_reduction_inside_a_step(be, mode, tokens, m, n, pitch):
+    test_reductions_of_any_length_end_inside_a_step(be, mode, tokens, m, n, pitch)
+
+
 @pytest.mark.parametrize("rows,kin,nout,layers", [(4096, 16, 512, 6), (4096, 384, 48, 5), (2048, 8, 256, 16)])
 def test_strided_batch_of_thin_weight_gradients_splits_the_reduction(be, rows, kin, nout, layers):
     """A batch of thin outputs over a long reduction (an adapter's rank x d gradients over the
