@@ -21,7 +21,9 @@ typedef unsigned int u32x4_s __attribute__((ext_vector_type(4)));
 
 
 // MB x NB blocks of 16 rows x 16 columns per workgroup.
-template <int MB, int NB, int WAVES, int CHUNK>
+// PLAIN: no activation in the store pass (whose code a call of a few rows would fetch for nothing: GELU is two thirds of
+// the kernel).
+template <int MB, int NB, int WAVES, int CHUNK, bool PLAIN>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(GemmArgs g) {
   extern __shared__ float skinny_red[];  // [WAVES][MB * NB][4][64]
   gemm_select_batch(g, blockIdx.z);
@@ -93,8 +95,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(GemmArgs g) {
       x[v] = part[0];
     }
     if (row < g.M && col < g.N)
-      bad |= g.epi == OMX_EPI_NONE ? gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3])
-                                   : gemm_store4_epi(g, 0, row, col, x[0], x[1], x[2], x[3]);
+      bad |= PLAIN ? gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3]) : gemm_store4_epi(g, 0, row, col, x[0], x[1], x[2], x[3]);
   }
   if (bad) dev_raise_fault(g.fault, g.tag);
 }
@@ -130,7 +131,8 @@ int skinny_tile(const GemmArgs& g, long units) {
 template <int MB, int NB, int WAVES>
 int32_t launch_skinny_waves(omx_ctx* ctx, const GemmArgs& g) {
   constexpr int smem = WAVES * MB * NB * 1024;
-  auto kernel = &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK>;
+  auto kernel = g.epi == OMX_EPI_NONE ? &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK, true>
+                                      : &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK, false>;
   if constexpr (smem > 64 * 1024)
     OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
   dim3 grid(static_cast<unsigned>((g.N + 16 * NB - 1) / (16 * NB)), static_cast<unsigned>((g.M + 16 * MB - 1) / (16 * MB)),

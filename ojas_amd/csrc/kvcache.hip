@@ -38,6 +38,7 @@ struct KvArgs {
   int batch, tq, heads, kv_heads, dim, capacity, group;
   long kv_len, window, read_lo;
   int tiles_per_block, nparts;
+  unsigned int read_slot;  // the ring's slot of position read_lo
   float scale;
   OmxFaultWord* fault;
   unsigned long long tag;
@@ -241,6 +242,10 @@ __global__ __launch_bounds__(64) void cached_attention_partial_kernel(KvArgs a) 
 // own keys and the groups are summed once, at the end of the block.
 constexpr int KG_ROUNDS = 16;
 constexpr int KG_ROWS = 4;  // query rows per block
+// Waves of a block with one row where blocks are few: sixteen of eight rounds (half the registers) over bf16 caches, eight
+// of sixteen over f32 ones, whose pieces would not fit the 128 registers a sixteen-wave block leaves each lane.
+template <typename T>
+constexpr int KG_FEW_WAVES = sizeof(T) == 2 ? 16 : 8;
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
@@ -265,14 +270,41 @@ __device__ __forceinline__ float across_groups(float v, F f) {
   return v;
 }
 
+// Four elements of a cache row as they sit in memory. `get<true>` is a point that no use of them moves ahead of.
+template <typename T>
+struct KvPiece {
+  float4 q;
+  __device__ __forceinline__ void load(const T* p) { q = *reinterpret_cast<const float4*>(p); }
+  template <bool HOLD>
+  __device__ __forceinline__ void get(float (&v)[4]) {
+    if constexpr (HOLD) asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(q.z), "+v"(q.w));
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+  }
+};
+template <>
+struct KvPiece<unsigned short> {
+  uint2 q;
+  __device__ __forceinline__ void load(const unsigned short* p) { q = *reinterpret_cast<const uint2*>(p); }
+  template <bool HOLD>
+  __device__ __forceinline__ void get(float (&v)[4]) {
+    if constexpr (HOLD) asm volatile("" : "+v"(q.x), "+v"(q.y));
+    v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u);
+    v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
+  }
+};
+
 // ROWS query rows per block: KG_ROWS, or one where a KV head has a single row (ungrouped heads, one new
-// token), which is a quarter of the code and half the registers. WAVES waves share a block's keys (a contiguous run each) and add up in LDS in wave order. When one block
+// token), which is a quarter of the code and half the registers. A call of few blocks runs every instruction about
+// once, so it is bound by fetching its own code and by one chain of memory latencies: positions are 32-bit offsets from
+// the tile, non-finite values are collected with one multiply-add each (x * 0 is NaN for them), and a single row
+// takes more waves of fewer rounds (KG_FEW_WAVES): 15.0 -> 5.3 KiB, 12 heads x 301 positions 12.1 -> 6.5 us.
+// WAVES waves share a block's keys (a contiguous run each) and add up in LDS in wave order. When one block
 // covers a row's whole span (nparts == 1) it writes the output itself: no partials in memory, no second launch.
-template <typename T, int LPK, int WAVES, int ROWS>
+template <typename T, int LPK, int WAVES, int ROWS, int ROUNDS>
 __global__ __launch_bounds__(WAVES * 64) void cached_attention_group_kernel(KvArgs a) {
   __shared__ float meet[WAVES][ROWS][LPK * 4 + 2];
   constexpr int G = 64 / LPK;               // keys per round
-  constexpr int TILE = KG_ROUNDS * G;       // keys per tile
+  constexpr int TILE = ROUNDS * G;       // keys per tile
   constexpr float LOG2E = 1.4426950408889634f;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int part = blockIdx.x, chunk = blockIdx.y;
@@ -281,18 +313,25 @@ __global__ __launch_bounds__(WAVES * 64) void cached_attention_group_kernel(KvAr
   constexpr int dim = LPK * 4;
   const int rows_all = a.tq * a.group;
   const int row0 = chunk * ROWS;
-  const int rows = min(ROWS, rows_all - row0);
+  const int rows = ROWS == 1 ? 1 : min(ROWS, rows_all - row0);
   bool bad = false;
+  float check[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // NaN once a value row that was read is not finite
 
   long p_of[ROWS], first_of[ROWS], out_row[ROWS];
   float q[ROWS][4];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    const int rr = min(row0 + r, rows_all - 1);
-    const int i = rr / a.group, h = kvh * a.group + (rr - i * a.group);
-    p_of[r] = a.kv_len - a.tq + i;
-    first_of[r] = a.window > 0 ? max(0l, p_of[r] + 1 - a.window) : 0l;
-    out_row[r] = (static_cast<long>(b) * a.tq + i) * a.heads + h;
+    if constexpr (ROWS == 1) {  // the only row: the last position, which sees every key that is read
+      p_of[r] = a.kv_len - 1;
+      first_of[r] = a.read_lo;
+      out_row[r] = static_cast<long>(b) * a.heads + kvh;
+    } else {
+      const int rr = min(row0 + r, rows_all - 1);
+      const int i = rr / a.group, h = kvh * a.group + (rr - i * a.group);
+      p_of[r] = a.kv_len - a.tq + i;
+      first_of[r] = a.window > 0 ? max(0l, p_of[r] + 1 - a.window) : 0l;
+      out_row[r] = (static_cast<long>(b) * a.tq + i) * a.heads + h;
+    }
     const float4 qv = *reinterpret_cast<const float4*>(a.q + out_row[r] * dim + d0);
     q[r][0] = qv.x; q[r][1] = qv.y; q[r][2] = qv.z; q[r][3] = qv.w;
     bad |= !(dev_finite(qv.x) && dev_finite(qv.y) && dev_finite(qv.z) && dev_finite(qv.w));
@@ -318,34 +357,48 @@ __global__ __launch_bounds__(WAVES * 64) void cached_attention_group_kernel(KvAr
   const long part_lo = block_lo + wave * wave_keys;
   const long part_hi = min(block_hi, part_lo + wave_keys);
   for (long pos0 = part_lo; pos0 < part_hi; pos0 += TILE) {
-    const int slot0 = static_cast<int>(pos0 % a.capacity);
-    float kv[KG_ROUNDS][4], vv[KG_ROUNDS][4];
+    const int left = static_cast<int>(min(static_cast<long>(TILE), part_hi - pos0));
+    // The span is within the capacity: a position wraps the ring at most once.
+    const unsigned int ahead = a.read_slot + static_cast<unsigned int>(pos0 - a.read_lo), capacity = a.capacity;
+    const unsigned int slot0 = ahead >= capacity ? ahead - capacity : ahead;
+    KvPiece<T> kr[ROUNDS], vr[ROUNDS];
 #pragma unroll
-    for (int i = 0; i < KG_ROUNDS; ++i) {
+    for (int i = 0; i < ROUNDS; ++i) {
       // Every lane loads, with no branch around the load, so that the compiler issues all 32
       // before it waits for the first: a key past the end of the part re-reads the tile's first
       // key (a slot this block reads anyway), and its weight below is exactly zero.
-      const int key = (pos0 + i * G + g < part_hi) ? i * G + g : 0;
-      int slot = slot0 + key;  // a tile wraps the ring at most once
-      slot = slot >= a.capacity ? slot - a.capacity : slot;
+      const int key = i * G + g < left ? i * G + g : 0;
+      unsigned int slot = slot0 + key;  // a tile wraps the ring at most once
+      slot = slot >= capacity ? slot - capacity : slot;
       const size_t off = static_cast<size_t>(((base_b + slot) * a.kv_heads + kvh) * dim + d0);
-      dev_load4(kc, off, kv[i]);
-      dev_load4(vc, off, vv[i]);
+      kr[i].load(kc + off);
+      vr[i].load(vc + off);
+    }
+    // Every load goes out before the first product (the compiler otherwise moves products up between them, each with
+    // its wait: 64 sequences of 1024 positions, 103 us instead of 73). Four rows have no registers to hold them all.
+    if constexpr (ROWS == 1) asm volatile("" ::: "memory");
+    float kv[ROUNDS][4], vv[ROUNDS][4];
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i) {
+      kr[i].template get<ROWS == 1>(kv[i]);
+      vr[i].template get<ROWS == 1>(vv[i]);
     }
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
       if (r < rows) {  // uniform
-        float s[KG_ROUNDS];
+        float s[ROUNDS];
         float tile_max = -INFINITY;
+        // The keys of this tile that the row sees: low <= offset <= high.
+        const int low = ROWS == 1 ? 0 : static_cast<int>(min(static_cast<long>(TILE), max(0l, first_of[r] - pos0)));
+        const int high = ROWS == 1 ? left - 1 : static_cast<int>(max(-1l, min(static_cast<long>(left - 1), p_of[r] - pos0)));
 #pragma unroll
-        for (int i = 0; i < KG_ROUNDS; ++i) {
+        for (int i = 0; i < ROUNDS; ++i) {
           float dot = q[r][0] * kv[i][0];
           dot = fmaf(q[r][1], kv[i][1], dot);
           dot = fmaf(q[r][2], kv[i][2], dot);
           dot = fmaf(q[r][3], kv[i][3], dot);
           dot = group_sum<LPK>(dot);
-          const long pos = pos0 + i * G + g;
-          const bool seen = pos < part_hi && pos <= p_of[r] && pos >= first_of[r];
+          const bool seen = i * G + g <= high && i * G + g >= low;
           const float sc = dot * scale2;
           bad |= seen && !dev_finite(sc);
           s[i] = seen ? sc : -INFINITY;
@@ -359,22 +412,29 @@ __global__ __launch_bounds__(WAVES * 64) void cached_attention_group_kernel(KvAr
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[r][e] *= corr;
 #pragma unroll
-          for (int i = 0; i < KG_ROUNDS; ++i) {
+          for (int i = 0; i < ROUNDS; ++i) {
             const float p = __builtin_amdgcn_exp2f(s[i] - m_new);  // 0 for a hidden key
             sum += p;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[r][e] = fmaf(p, vv[i][e], acc[r][e]);
+            for (int e = 0; e < 4; ++e) {
+              acc[r][e] = fmaf(p, vv[i][e], acc[r][e]);
+              if constexpr (ROWS == 1) check[e] = fmaf(vv[i][e], 0.0f, check[e]);
+            }
           }
           l[r] = l[r] * corr + sum;  // this lane group's keys only
           m[r] = m_new;
         }
       }
     }
+    // (a single row sees every key that is read: one that is not finite shows in its score)
+    if constexpr (ROWS > 1) {
 #pragma unroll
-    for (int i = 0; i < KG_ROUNDS; ++i)
-      bad |= !(dev_finite(kv[i][0]) && dev_finite(kv[i][1]) && dev_finite(kv[i][2]) && dev_finite(kv[i][3]) &&
-               dev_finite(vv[i][0]) && dev_finite(vv[i][1]) && dev_finite(vv[i][2]) && dev_finite(vv[i][3]));
+      for (int i = 0; i < ROUNDS; ++i)
+        bad |= !(dev_finite(kv[i][0]) && dev_finite(kv[i][1]) && dev_finite(kv[i][2]) && dev_finite(kv[i][3]) &&
+                 dev_finite(vv[i][0]) && dev_finite(vv[i][1]) && dev_finite(vv[i][2]) && dev_finite(vv[i][3]));
+    }
   }
+  if constexpr (ROWS == 1) bad |= !(check[0] == 0.0f && check[1] == 0.0f && check[2] == 0.0f && check[3] == 0.0f);
 
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
@@ -405,8 +465,11 @@ __global__ __launch_bounds__(WAVES * 64) void cached_attention_group_kernel(KvAr
       total = fmaf(meet[w][r][dim + 1], weight, total);
       sum = fmaf(meet[w][r][d], weight, sum);
     }
-    const int rr = row0 + r, i = rr / a.group;
-    const long out_at = (static_cast<long>(b) * a.tq + i) * a.heads + kvh * a.group + (rr - i * a.group);
+    long out_at = out_row[0];
+    if constexpr (ROWS > 1) {
+      const int rr = row0 + r, i = rr / a.group;
+      out_at = (static_cast<long>(b) * a.tq + i) * a.heads + kvh * a.group + (rr - i * a.group);
+    }
     if (a.nparts == 1) {
       bad |= !(dev_finite(total) && total > 0.0f);
       a.out[out_at * dim + d] = sum * (1.0f / total);
@@ -472,20 +535,19 @@ __device__ __forceinline__ bool kv_finite(const float* p) {
     return dev_finite(*p);
   }
 }
-template <typename T, int VEC>
-__device__ __forceinline__ void kv_put(const KvWrite& w, size_t i) {
-  size_t row, b;
-  if (w.n <= 0xffffffffull) {  // 32-bit divisions where they do
-    row = static_cast<unsigned int>(i) / w.step;
-    b = static_cast<unsigned int>(row) / w.tn;
-  } else {
-    row = i / w.step;
-    b = row / w.tn;
-  }
+// Where element i of src goes.
+template <typename T, typename Index>
+__device__ __forceinline__ T* kv_place(const KvWrite& w, Index i) {
+  const Index row = i / w.step, b = row / w.tn;
   const unsigned int e = static_cast<unsigned int>(i - row * w.step);
   const unsigned int j = static_cast<unsigned int>(row - b * w.tn);
   const unsigned int slot = w.at + j < w.capacity ? w.at + j : w.at + j - w.capacity;  // at < capacity, tn <= capacity
-  T* dst = static_cast<T*>(w.cache) + (b * w.capacity + slot) * w.step + e;
+  return static_cast<T*>(w.cache) + (static_cast<size_t>(b) * w.capacity + slot) * w.step + e;
+}
+template <typename T, int VEC>
+__device__ __forceinline__ void kv_put(const KvWrite& w, size_t i) {
+  // (32-bit divisions where they do)
+  T* dst = w.n <= 0xffffffffull ? kv_place<T>(w, static_cast<unsigned int>(i)) : kv_place<T>(w, i);
   if constexpr (VEC == 4) {
     float v[4];
     dev_load4(w.src, i, v);
@@ -500,23 +562,35 @@ __device__ __forceinline__ void kv_put(const KvWrite& w, size_t i) {
 // channels: at 49152 values the scan alone is 10 us, and two launches are ahead from some 16384 on.
 constexpr size_t KV_ONE_LAUNCH = 1u << 14;
 constexpr int KV_SCAN_THREADS = 1024;
+// A thread writes at most one piece, which it loads first: one workgroup (4096 values) has scanned everything with that.
 template <typename T, int VEC>
 __global__ __launch_bounds__(KV_SCAN_THREADS) void kv_scan_write_kernel(KvWrite w) {
-  bool bad = false;
-  constexpr size_t STRIDE = KV_SCAN_THREADS * VEC;
-  for (size_t i0 = static_cast<size_t>(threadIdx.x) * VEC; i0 < w.n; i0 += 8 * STRIDE) {
+  constexpr unsigned int STRIDE = KV_SCAN_THREADS * VEC;
+  const unsigned int n = static_cast<unsigned int>(w.n), own = (blockIdx.x * KV_SCAN_THREADS + threadIdx.x) * VEC;
+  float v[VEC];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {  // eight loads in flight; past the end the last piece again
-      const size_t i = i0 + u * STRIDE;
-      bad |= !kv_finite<VEC>(w.src + (i < w.n ? i : w.n - VEC));
-    }
+  for (int e = 0; e < VEC; ++e) v[e] = 0.0f;
+  T* dst = nullptr;
+  if (own < n) {
+    if constexpr (VEC == 4) dev_load4(w.src, own, v);
+    else v[0] = w.src[own];
+    dst = kv_place<T>(w, own);
+  }
+  bool bad = false;
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) bad |= !dev_finite(v[e]);
+  if (gridDim.x > 1) {
+#pragma unroll 4
+    for (unsigned int i = threadIdx.x * VEC; i < n; i += STRIDE) bad |= !kv_finite<VEC>(w.src + i);
   }
   if (__syncthreads_or(bad)) {
     if (bad) dev_raise_fault(w.fault, w.tag);
     return;
   }
-  for (size_t i = (static_cast<size_t>(blockIdx.x) * KV_SCAN_THREADS + threadIdx.x) * VEC; i < w.n; i += gridDim.x * STRIDE)
-    kv_put<T, VEC>(w, i);
+  if (own < n) {
+    if constexpr (VEC == 4) dev_store4(dst, 0, v);
+    else dev_store(dst, 0, v[0]);
+  }
 }
 // A longer one: the first launch scans, the second copies unless the scan refused. The word between them
 // holds the tag of a refused scan, which no other call shares, so nothing has to be cleared.
@@ -553,15 +627,15 @@ int32_t launch_kv_write(omx_ctx* ctx, const KvWrite& w) {
 
 template <typename T, int LPK, int NPL>
 int32_t launch_group(omx_ctx* ctx, const KvArgs& a, dim3 grid, long rows_total, int waves) {
-  auto go = [&](auto eight, auto four, auto one) {
-    omx_launch(ctx, (waves == 8 ? eight : waves == 4 ? four : one), grid, dim3(waves * 64), 0, a);
+  auto go = [&](auto most, auto four, auto one) {
+    omx_launch(ctx, (waves >= 8 ? most : waves == 4 ? four : one), grid, dim3(waves * 64), 0, a);
   };
   if (a.tq * a.group == 1)
-    go(&cached_attention_group_kernel<T, LPK, 8, 1>, &cached_attention_group_kernel<T, LPK, 4, 1>,
-       &cached_attention_group_kernel<T, LPK, 1, 1>);
+    go(&cached_attention_group_kernel<T, LPK, KG_FEW_WAVES<T>, 1, 8 * KG_ROUNDS / KG_FEW_WAVES<T>>, &cached_attention_group_kernel<T, LPK, 4, 1, KG_ROUNDS>,
+       &cached_attention_group_kernel<T, LPK, 1, 1, KG_ROUNDS>);
   else
-    go(&cached_attention_group_kernel<T, LPK, 8, KG_ROWS>, &cached_attention_group_kernel<T, LPK, 4, KG_ROWS>,
-       &cached_attention_group_kernel<T, LPK, 1, KG_ROWS>);
+    go(&cached_attention_group_kernel<T, LPK, 8, KG_ROWS, KG_ROUNDS / 2>, &cached_attention_group_kernel<T, LPK, 4, KG_ROWS, KG_ROUNDS>,
+       &cached_attention_group_kernel<T, LPK, 1, KG_ROWS, KG_ROUNDS>);
   OMX_LAUNCH_CHECK(ctx, "cached_attention_group_kernel");
   if (a.nparts == 1) return OMX_OK;
   omx_launch(ctx, (cached_attention_merge_kernel<NPL>), dim3(static_cast<unsigned>(rows_total)), dim3(64), 0, a, rows_total);
@@ -665,6 +739,7 @@ int32_t omx_cached_attention_forward(omx_ctx* ctx, const void* q, const void* k_
   a.kv_len = static_cast<long>(kv_len);
   a.window = static_cast<long>(window);
   a.read_lo = static_cast<long>(kv_len - span);
+  a.read_slot = static_cast<unsigned int>((kv_len - span) % capacity);
   a.scale = 1.0f / std::sqrt(static_cast<float>(head_dim));
   a.fault = ctx->fault;
   a.tag = omx_tag(ctx, F_CACHED_ATTENTION);
@@ -680,10 +755,10 @@ int32_t omx_cached_attention_forward(omx_ctx* ctx, const void* q, const void* k_
   const uint64_t groups = batch * kv_heads * chunks;
   uint64_t waves = 1, parts;
   if (grouped) {
-    // Few blocks take eight waves each (they share the keys and meet in LDS), a few thousand fill the chip
+    // Few blocks take eight or sixteen waves each (they share the keys and meet in LDS), a few thousand fill the chip
     // with one. A row's keys are split over blocks, with partials in memory and a merge launch, only
     // when there are not waves enough and every wave still has a tile of 64 keys.
-    waves = groups <= static_cast<uint64_t>(ctx->cu_count) ? 8 : groups <= 4ull * ctx->cu_count ? 4 : 1;
+    waves = groups <= static_cast<uint64_t>(ctx->cu_count) ? (rows_per_group > 1 ? 8 : bf16 ? KG_FEW_WAVES<unsigned short> : KG_FEW_WAVES<float>) : groups <= 4ull * ctx->cu_count ? 4 : 1;
     parts = std::min<uint64_t>((8ull * ctx->cu_count + groups * waves - 1) / (groups * waves), (tiles + waves - 1) / waves);
   } else {
     // Enough blocks to fill the chip several times over, but no more parts than tiles.

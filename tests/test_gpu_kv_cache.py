@@ -203,3 +203,32 @@ def test_prompt_chunks_on_the_matrix_units(be, b, tq, h, hkv, d, capacity, kv_le
     dk, dv = (be.upload(x, BF16) if bf16_cache else be.upload(x) for x in (k, v))
     got = be.download(be.cached_attention_forward(be.upload(q), dk, dv, kv_len, window))
     assert np.abs(got - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))
+
+
+@pytest.mark.parametrize("b,h,d,capacity,kv_len,window", [
+    (1, 3, 64, 1, 1, None), (1, 3, 64, 40, 500, 37), (1, 2, 64, 512, 512, None), (2, 2, 64, 513, 1300, 513), (1, 2, 128, 300, 299, None),
+    (1, 1, 256, 140, 1000, 131), (3, 2, 16, 70, 2100, 66), (1, 2, 4, 3000, 2500, None)])
+@pytest.mark.parametrize("bf16_cache", [False, True])
+def test_one_row_of_few_blocks(be, b, h, d, capacity, kv_len, window, bf16_cache):
+    """One new token of ungrouped heads in few blocks (sixteen waves over a bf16 cache, eight over an f32 one): fewer keys
+    than waves, a wave's tile exactly full and one key more, rings that wrap inside a wave's keys; a key or a value
+    that is not finite raises, one outside the window does not."""
+    r = np.random.default_rng(kv_len + d)
+    q = r.standard_normal((b, 1, h, d)).astype(np.float32)
+    seq = [r.standard_normal((b, kv_len, h, d)).astype(np.float32) for _ in range(2)]
+    if bf16_cache:
+        seq = [orc.round_bf16(x) for x in seq]
+    k, v = (ring(x, capacity, kv_len, np.nan) for x in seq)
+    if window:
+        for j in range(max(0, kv_len - capacity), kv_len - window):  # nothing reads these
+            k[:, j % capacity] = v[:, j % capacity] = np.nan
+    up = lambda x: be.upload(x, BF16) if bf16_cache else be.upload(x)
+    want = orc.cached_attention_forward(q, np.nan_to_num(k), np.nan_to_num(v), kv_len, window or 0)
+    got = be.download(be.cached_attention_forward(be.upload(q), up(k), up(v), kv_len, window))
+    assert np.abs(got - want).max() <= 1e-5 * max(1.0, float(np.abs(want).max()))
+    for which in (0, 1):
+        broken = [k.copy(), v.copy()]
+        broken[which][-1, (kv_len - 1) % capacity, -1, -1] = np.inf
+        be.cached_attention_forward(be.upload(q), up(broken[0]), up(broken[1]), kv_len, window)
+        with pytest.raises(OjasError):
+            be.sync()
