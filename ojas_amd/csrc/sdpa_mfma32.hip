@@ -1,5 +1,6 @@
 // f32 attention on the f32 matrix instructions (v_mfma_f32_16x16x4_f32), head dims 16 / 32 / 64 / 128: causal SDPA
-// forward and backward of the f32 tier and the attention of a prompt chunk over a KV cache.
+// forward and backward of the f32 tier and the attention of a prompt chunk over a KV cache (over bf16 caches of head dim
+// 64 and 128 on the bf16 ones, sdpa_prompt_kernel).
 //
 // Reference: ojas-cpu/src/attn.rs (causal_sdpa_*; trait ojas-core/src/backend.rs:1729-1792) and
 // ojas-cpu/src/kv.rs (cached_attention_forward, backend.rs:2526-2555). Same formulas as sdpa.hip's row
@@ -306,6 +307,249 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   if (bad) dev_raise_fault(a.fault, a.tag);
 }
 
+// ---------------------------------------------------------------- forward over bf16 caches
+// Keys and values are bf16 there, so the bf16 matrix instructions (sixteen times the f32 rate) multiply them exactly;
+// the f32 operand beside them, a query or a probability, is cut into three bf16 parts that hold all of its 24 bits
+// (each cut is exact), and the three products are added up in f32, smallest first. Every product is exact, as on the
+// f32 instructions, and a row's sums have half as many roundings; three sixteenths of the matrix time.
+//
+// A workgroup takes 16 MB rows and its four waves share the keys, AtPrompt::KEYS at a time. No wave reads another's
+// keys, so keys go from memory straight into fragments and only values pass through LDS, a region per wave, where
+// the transposing reads form the other operand: no barrier before the waves meet. The next keys and values are on
+// their way during softmax and the second product. Bound by vector instructions: softmax and the cuts.
+// us on f32 instructions -> here (relative error against 64 bits): 4 x 12 heads x 64, 256 new positions of 700: 38.6 -> 20.6
+// (2.5e-7 -> 1.5e-7); 8 x 16 over 4 KV heads x 64, 512 of 1024: 173 -> 85 (5.2e-7 -> 1.6e-7); 2 x 8 over 2 x 128, 100 of 800:
+// 41 -> 16 (2.9e-7 -> 1.7e-7).
+typedef __bf16 bf16x8_a __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4_a __attribute__((ext_vector_type(4)));
+typedef short short4_a __attribute__((ext_vector_type(4)));
+
+struct AtParts {
+  u32x4_a part[3];  // largest first
+  __device__ __forceinline__ void cut(const float (&x)[8]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      float a = x[2 * p], b = x[2 * p + 1];
+#pragma unroll
+      for (int n = 0; n < 3; ++n) {
+        const unsigned int wa = __float_as_uint(a), wb = __float_as_uint(b);
+        part[n][p] = __builtin_amdgcn_perm(wb, wa, 0x07060302u);  // the upper halves, a's below b's
+        a -= __uint_as_float(wa & 0xffff0000u);
+        b -= __uint_as_float(wb & 0xffff0000u);
+      }
+    }
+  }
+};
+// acc += A . (the parts), A's lane values 8 g + j beside theirs.
+__device__ __forceinline__ floatx4_a at_mfma_parts(u32x4_a a, const AtParts& b, floatx4_a acc) {
+#pragma unroll
+  for (int n = 2; n >= 0; --n)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_a, a), __builtin_bit_cast(bf16x8_a, b.part[n]), acc, 0, 0, 0);
+  return acc;
+}
+
+template <int D>
+struct AtPrompt {
+  static constexpr int KEYS = 4096 / D;      // per wave and step
+  static constexpr int NB = KEYS / 16;       // blocks of 16 keys
+  static constexpr int KS = D / 32, DB = D / 16;
+  static constexpr int PITCH = 2 * D + 32;   // bytes of a value row in LDS: eight rows' 32-byte pieces in distinct banks
+  static constexpr int PIECES = KEYS * D / 8 / 64;
+};
+
+// (three workgroups per compute unit with one block of rows: 168 registers)
+template <int D, int MB>
+__global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_prompt_kernel(Sdpa32Args a) {
+  using X = AtPrompt<D>;
+  __shared__ __align__(16) char lds[4 * X::KEYS * X::PITCH];
+  static_assert(512 + 4 * X::DB * 1024 <= 4 * X::KEYS * X::PITCH, "the waves' sums fit");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const int rows = a.tq * a.rep;
+  const int r0 = (gridDim.x - 1 - blockIdx.x) * (16 * MB);  // the rows that see the most keys first
+  AtRow at[MB];
+  AtParts q[MB][X::KS];
+  int pos[MB], low[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const int r = r0 + m * 16 + i;
+    at[m] = at_unpack(min(r, rows - 1), a.rep);
+    const float* row = a.q + b * a.q_b + (static_cast<long>(kvh) * a.rep + at[m].head) * a.q_h + static_cast<long>(at[m].query) * a.q_t;
+#pragma unroll
+    for (int s = 0; s < X::KS; ++s) {
+      const float4 x = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g), y = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g + 4);
+      const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+      q[m][s].cut(v);
+    }
+    pos[m] = r < rows ? a.q_pos0 + at[m].query : -1;
+    low[m] = a.window > 0 ? max(0, pos[m] + 1 - a.window) : 0;
+  }
+  const int first_pos = a.q_pos0 + at_unpack(r0, a.rep).query;
+  const int last_pos = a.q_pos0 + at_unpack(min(r0 + 16 * MB, rows) - 1, a.rep).query;
+  const int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / X::KEYS, t_last = last_pos / X::KEYS;
+  const unsigned short* kb = static_cast<const unsigned short*>(a.k) + b * a.k_b + kvh * a.k_h;
+  const unsigned short* vb = static_cast<const unsigned short*>(a.v) + b * a.k_b + kvh * a.k_h;
+  char* region = lds + wave * (X::KEYS * X::PITCH);
+
+  u32x4_a kn[X::NB][X::KS], vn[X::PIECES];
+  auto slot_at = [&](int key) {
+    int slot = a.slot0 + key;  // a ring wraps at most once over the keys that are read
+    return static_cast<long>(slot >= a.capacity ? slot - a.capacity : slot) * a.k_t;
+  };
+  auto fetch = [&](int t) {  // keys past the last one are rows of zeros
+#pragma unroll
+    for (int n = 0; n < X::NB; ++n) {
+      const int key = t * X::KEYS + n * 16 + i;
+#pragma unroll
+      for (int s = 0; s < X::KS; ++s) {
+        if (key < a.tk) kn[n][s] = *reinterpret_cast<const u32x4_a*>(kb + slot_at(key) + 32 * s + 8 * g);
+        else kn[n][s] = u32x4_a{0u, 0u, 0u, 0u};
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < X::PIECES; ++p) {
+      const int idx = lane + 64 * p, key = t * X::KEYS + idx / (D / 8);
+      if (key < a.tk) vn[p] = *reinterpret_cast<const u32x4_a*>(vb + slot_at(key) + idx % (D / 8) * 8);
+      else vn[p] = u32x4_a{0u, 0u, 0u, 0u};
+    }
+  };
+
+  const float scale2 = a.scale * AT_LOG2E;
+  floatx4_a o[MB][X::DB];
+  float mx[MB], sum[MB];  // in the exp2 domain; `sum` over this lane's keys only
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    mx[m] = -INFINITY;
+    sum[m] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < X::DB; ++d) o[m][d] = at_zero();
+  }
+  bool bad = false;
+  if (t_first + wave <= t_last) fetch(t_first + wave);
+  for (int t = t_first + wave; t <= t_last; t += 4) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the previous values have been read
+#pragma unroll
+    for (int p = 0; p < X::PIECES; ++p) {
+      const int idx = lane + 64 * p;
+      *reinterpret_cast<u32x4_a*>(region + idx / (D / 8) * X::PITCH + idx % (D / 8) * 16) = vn[p];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    floatx4_a s[MB][X::NB];
+#pragma unroll
+    for (int n = 0; n < X::NB; ++n)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        s[m][n] = at_zero();
+#pragma unroll
+        for (int ks = 0; ks < X::KS; ++ks) s[m][n] = at_mfma_parts(kn[n][ks], q[m][ks], s[m][n]);
+      }
+    if (t + 4 <= t_last) fetch(t + 4);
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      float top = -INFINITY;
+#pragma unroll
+      for (int n = 0; n < X::NB; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int key = t * X::KEYS + n * 16 + 4 * g + v;
+          const bool seen = key <= pos[m] && key >= low[m];
+          const float x = s[m][n][v] * scale2;
+          bad |= seen && !dev_finite(x);
+          s[m][n][v] = seen ? x : -INFINITY;
+          top = fmaxf(top, s[m][n][v]);
+        }
+      top = at_row_max(top);
+      const float mx_new = fmaxf(mx[m], top), base = mx_new == -INFINITY ? 0.0f : mx_new;
+      const float rescale = __builtin_amdgcn_exp2f(mx[m] - base);
+      mx[m] = mx_new;
+      sum[m] *= rescale;
+#pragma unroll
+      for (int d = 0; d < X::DB; ++d)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[m][d][v] *= rescale;
+#pragma unroll
+      for (int n = 0; n < X::NB; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          s[m][n][v] = __builtin_amdgcn_exp2f(s[m][n][v] - base);
+          sum[m] += s[m][n][v];
+        }
+    }
+    // 32 keys at a time: a lane's eight are 4 g + v of two blocks, and so are the transposed values'.
+#pragma unroll
+    for (int h = 0; h < X::NB / 2; ++h) {
+      AtParts p[MB];
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        const float x[8] = {s[m][2 * h][0], s[m][2 * h][1], s[m][2 * h][2], s[m][2 * h][3],
+                            s[m][2 * h + 1][0], s[m][2 * h + 1][1], s[m][2 * h + 1][2], s[m][2 * h + 1][3]};
+        p[m].cut(x);
+      }
+#pragma unroll
+      for (int d = 0; d < X::DB; ++d) {
+        typedef short4_a __attribute__((address_space(3))) * lds_ptr;
+        char* at_v = region + (32 * h + 4 * g + (i >> 2)) * X::PITCH + 32 * d + (i & 3) * 8;
+        const short4_a lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at_v));
+        const short4_a hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at_v + 16 * X::PITCH));
+        const uint2 l = __builtin_bit_cast(uint2, lo), u = __builtin_bit_cast(uint2, hi);
+        const u32x4_a value = {l.x, l.y, u.x, u.y};
+#pragma unroll
+        for (int m = 0; m < MB; ++m) o[m][d] = at_mfma_parts(value, p[m], o[m][d]);
+      }
+    }
+  }
+  // The four waves' shares of the same rows: wave w adds up the column blocks w, w + 4, ...
+  float* stat = reinterpret_cast<float*>(lds);                // [4][2][16]
+  float4* part = reinterpret_cast<float4*>(lds + 512);        // [4][DB][64]
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const float all_keys = at_row_sum(sum[m]);
+    __syncthreads();
+    if (g == 0) {
+      stat[wave * 32 + i] = mx[m];
+      stat[wave * 32 + 16 + i] = all_keys;
+    }
+#pragma unroll
+    for (int d = 0; d < X::DB; ++d) part[(wave * X::DB + d) * 64 + lane] = make_float4(o[m][d][0], o[m][d][1], o[m][d][2], o[m][d][3]);
+    __syncthreads();
+    float all = -INFINITY, weight[4], total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) all = fmaxf(all, stat[w * 32 + i]);
+    const float base = all == -INFINITY ? 0.0f : all;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      weight[w] = __builtin_amdgcn_exp2f(stat[w * 32 + i] - base);
+      total = fmaf(weight[w], stat[w * 32 + 16 + i], total);
+    }
+    if (r0 + m * 16 + i < rows) {
+      bad |= !(dev_finite(total) && total > 0.0f);
+      const float f = 1.0f / total;
+      float* out = a.out + b * a.o_b + (static_cast<long>(kvh) * a.rep + at[m].head) * a.o_h + static_cast<long>(at[m].query) * a.o_t;
+#pragma unroll
+      for (int d0 = 0; d0 < X::DB; d0 += 4) {
+        float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float4 y = part[(w * X::DB + d0 + wave) * 64 + lane];
+          x[0] = fmaf(weight[w], y.x, x[0]);
+          x[1] = fmaf(weight[w], y.y, x[1]);
+          x[2] = fmaf(weight[w], y.z, x[2]);
+          x[3] = fmaf(weight[w], y.w, x[3]);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          x[v] *= f;
+          bad |= !dev_finite(x[v]);
+        }
+        *reinterpret_cast<float4*>(out + (d0 + wave) * 16 + 4 * g) = make_float4(x[0], x[1], x[2], x[3]);
+      }
+    }
+  }
+  if (bad) dev_raise_fault(a.fault, a.tag);
+}
+
 // ---------------------------------------------------------------- backward
 // p and dS of one lane's four scores, from the score and dP accumulators.
 struct AtGrad {
@@ -560,14 +804,30 @@ bool at_narrow(omx_ctx* ctx, long planes, long rows) { return planes * ((rows + 
 template <int D>
 int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) {
   const long rows = static_cast<long>(a.tq) * a.rep;
+  if constexpr (D >= 64) {
+    if (bf16_cache) {  // (attention over a cache has no lse)
+      // Twice the rows on a key's way only where half as many workgroups still fill the chip.
+      const bool two = D == 64 && (rows + 31) / 32 * planes >= 4l * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+      const long per = two ? 32 : 16;
+      dim3 blocks(static_cast<unsigned>((rows + per - 1) / per), planes);
+      if constexpr (D == 64) {
+        if (two) omx_launch(ctx, (sdpa_prompt_kernel<D, 2>), blocks, dim3(AT_THREADS), 0, a);
+      }
+      if (!two) omx_launch(ctx, (sdpa_prompt_kernel<D, 1>), blocks, dim3(AT_THREADS), 0, a);
+      OMX_LAUNCH_CHECK(ctx, "sdpa_prompt_kernel");
+      return OMX_OK;
+    }
+  }
   const bool narrow = at_narrow(ctx, planes, rows);
   const long bq = narrow ? 16 : 64;
   dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
+  using Cache = std::conditional_t<(D < 64), unsigned short, float>;  // bf16 caches of wider heads are gone by now
+  auto launch_bf16 = [&](auto kernel) { omx_launch(ctx, kernel, grid, dim3(AT_THREADS), 0, a); };
   if (narrow) {
-    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, unsigned short>), grid, dim3(AT_THREADS), 0, a);
+    if (bf16_cache) launch_bf16(&sdpa32_fwd_kernel<D, 4, Cache>);
     else omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, float>), grid, dim3(AT_THREADS), 0, a);
   } else {
-    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, unsigned short>), grid, dim3(AT_THREADS), 0, a);
+    if (bf16_cache) launch_bf16(&sdpa32_fwd_kernel<D, 1, Cache>);
     else omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, float>), grid, dim3(AT_THREADS), 0, a);
   }
   OMX_LAUNCH_CHECK(ctx, "sdpa32_fwd_kernel");

@@ -232,3 +232,24 @@ def test_one_row_of_few_blocks(be, b, h, d, capacity, kv_len, window, bf16_cache
         be.cached_attention_forward(be.upload(q), up(broken[0]), up(broken[1]), kv_len, window)
         with pytest.raises(OjasError):
             be.sync()
+
+
+@pytest.mark.parametrize("b,tq,h,hkv,d,capacity,kv_len,window", [
+    (1, 16, 1, 1, 64, 16, 16, None), (1, 17, 2, 2, 128, 33, 33, None), (2, 16, 3, 3, 64, 65, 400, 49), (1, 65, 4, 2, 128, 257, 257, None),
+    (32, 40, 16, 16, 64, 80, 77, None), (16, 33, 16, 8, 64, 100, 200, 60)])
+def test_prompt_chunks_over_bf16_caches_lose_nothing(be, b, tq, h, hkv, d, capacity, kv_len, window):
+    """The f32 operands in three bf16 parts, against 64-bit sums: one and two blocks of 16 rows per workgroup, keys that end
+    inside a block, rings and windows. A score has d + 1 roundings and a sum over kv_len keys that many: 1e-6 of the
+    result's norm is some four times what the f32 instructions showed over these lengths."""
+    r = np.random.default_rng(tq * 3 + d)
+    q = r.standard_normal((b, tq, h, d)).astype(np.float32)
+    seq = [orc.round_bf16(r.standard_normal((b, kv_len, hkv, d)).astype(np.float32)) for _ in range(2)]
+    k, v = (ring(x, capacity, kv_len, 0.0) for x in seq)
+    wide = [np.repeat(x.astype(np.float64), h // hkv, axis=2).transpose(0, 2, 1, 3) for x in seq]
+    s = q.astype(np.float64).transpose(0, 2, 1, 3) @ wide[0].transpose(0, 1, 3, 2) / np.sqrt(d)
+    at, key = kv_len - tq + np.arange(tq)[:, None], np.arange(kv_len)[None, :]
+    s = np.where((key <= at) & (key > at - (window or kv_len)), s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = ((p / p.sum(-1, keepdims=True)) @ wide[1]).transpose(0, 2, 1, 3)
+    got = be.download(be.cached_attention_forward(be.upload(q), be.upload(k, BF16), be.upload(v, BF16), kv_len, window))
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
