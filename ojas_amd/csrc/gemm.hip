@@ -601,7 +601,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
         dma_variant = 3;
       }
       // A few hundred to a few thousand tokens, or a model some hundred wide, make less than a round or two of those
-      // tiles. Two smaller ones in 64-column steps (whole cache lines of a k-contiguous row, three stages), where
+      // tiles. Two smaller ones in 64-column steps (whole cache lines of a k-contiguous row), where
       // they take a tenth less than the choice above, or a fifth less than the few-row kernel, whose
       // workgroups have all of cold weights in flight at once:
       //   7  128 x 64, four waves, two workgroups per compute unit;

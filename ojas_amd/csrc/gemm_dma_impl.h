@@ -7,6 +7,17 @@
 
 namespace {
 
+// Waits until at most `groups` (up to G) groups of LPS loads are still in flight.
+template <int G, int LPS>
+__device__ __forceinline__ void wait_loads(int groups) {
+  if constexpr (G <= 0) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+  } else {
+    if (groups >= G) __builtin_amdgcn_s_waitcnt(vmcnt_only(G * LPS));
+    else wait_loads<G - 1, LPS>(groups);
+  }
+}
+
 // EPI: the store pass (OMX_EPI_*). A kernel of its own per store pass keeps each one's code (a few KiB of
 // straight-line stores) and registers out of the others. TAIL: see StepBase.
 template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI, bool TAIL = false>
@@ -90,12 +101,8 @@ gemm_dma_kernel(GemmArgs g) {
     for (int t = 0; t < TN; ++t) b_off[t][kk] = A_BYTES + frag_offset<B_KM, BN, DBK>((wn * TN + t) * 32, kk, lane);
   }
   // Waits until at most `groups` of this wave's per-step load groups are still in flight.
-  auto wait_groups = [&](int groups) {
-    static_assert(2 * LPS < 64, "vmcnt is six bits");
-    if (groups >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * LPS));
-    else if (groups == 1) __builtin_amdgcn_s_waitcnt(vmcnt_only(LPS));
-    else __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-  };
+  static_assert((NST - 2) * LPS < 64, "vmcnt is six bits");
+  auto wait_groups = [&](int groups) { wait_loads<NST - 2, LPS>(groups); };
 
 #pragma unroll
   for (int i = 0; i < NST - 1; ++i)
@@ -261,7 +268,8 @@ int32_t launch_dma(omx_ctx* ctx, const GemmArgs& g) {
 
 // The tilings the dispatcher chooses among: 9 and 10: 256 x 256 and 256 x 192, one wave per SIMD, one
 // workgroup per compute unit (gemm_w4_impl.h); 3: 256 x 128 in 32-column steps (three stages, two workgroups per
-// compute unit); 6: 128 x 128 with four waves (three per compute unit).
+// compute unit); 6: 128 x 128 with four waves (three per compute unit); 7 and 8: 128 x 64 and 64 x 64 with four waves in
+// 64-column steps (two and three per compute unit).
 template <bool A_KM, bool B_KM>
 int32_t launch_variant(omx_ctx* ctx, const GemmArgs& g, int variant) {
   if (variant == 9 || variant == 10) {
@@ -272,8 +280,16 @@ int32_t launch_variant(omx_ctx* ctx, const GemmArgs& g, int variant) {
     return omx_fail(ctx, OMX_SHAPE, "gemm: no one-wave-per-SIMD kernel for this operand layout");
   }
   if (variant == 6) return launch_dma<A_KM, B_KM, 2, 2, 2, 2, 32, 3>(ctx, g);
-  if (variant == 7) return launch_dma<A_KM, B_KM, 2, 2, 2, 1, 64, 3>(ctx, g);
-  if (variant == 8) return launch_dma<A_KM, B_KM, 2, 2, 1, 1, 64, 3>(ctx, g);
+  // Up to one tile per compute unit nothing shares its LDS and a step waits for memory: five or six stages, some 90 KiB on
+  // their way. What counts is operands as a step or a decoder's pass finds them, out of the last cache or HBM: a prompt
+  // chunk of 1024 rows through 12 layers of d = 768: 9.9 -> 8.6 us per product; a step of 3500 tokens at d = 512: 2.51 ->
+  // 2.50 ms with 128 x 64 tiles that deep (2.43 against 2.45 before either). Repeated out of L2 short reductions take
+  // 0.6 us longer, 4096 columns 1.5 us less.
+  const bool alone = static_cast<long>(g.tiles_m) * g.tiles_n * g.splits * g.batches <= (ctx->cu_count > 0 ? ctx->cu_count : 256);
+  if (variant == 7)
+    return alone ? launch_dma<A_KM, B_KM, 2, 2, 2, 1, 64, 5>(ctx, g) : launch_dma<A_KM, B_KM, 2, 2, 2, 1, 64, 3>(ctx, g);
+  if (variant == 8)
+    return alone ? launch_dma<A_KM, B_KM, 2, 2, 1, 1, 64, 6>(ctx, g) : launch_dma<A_KM, B_KM, 2, 2, 1, 1, 64, 3>(ctx, g);
   return launch_dma<A_KM, B_KM, 4, 2, 2, 2, 32, 3>(ctx, g);
 }
 
