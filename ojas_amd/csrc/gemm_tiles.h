@@ -52,8 +52,7 @@ struct StepBase {
   // it (vmcnt(0) right after the issue), which serialises the loads with the products.
   template <int IMM>
   __device__ __forceinline__ void load(unsigned off, unsigned lds) const {
-    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(at), "s"(lds), "n"(IMM)
-                 : "memory", "scc");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(at), "s"(lds + IMM) : "memory");
   }
 };
 template <>

@@ -77,9 +77,28 @@ __global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __res
   bool bad = false;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    if constexpr (!TOGETHER) load(j);
-    xr[j].get(xv[j]);
-    if (add) {
+    if constexpr (!TOGETHER) {  // widened as they arrive (8192 rows of 2048: 38.8 us, 41.2 from waiting registers)
+      const int c = j * 256 + lane * 4;
+      if (c < dim) {
+        dev_load4<TX>(x, base + c, xv[j]);
+        if (add) {
+          float av[4];
+          dev_load4<TA>(add, base + c, av);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            xv[j][e] = xv[j][e] + av[e];
+            bad |= !dev_finite(xv[j][e]);
+          }
+          dev_store4<float>(sum_out, base + c, xv[j]);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv[j][e] = 0.0f;
+      }
+    } else {
+      xr[j].get(xv[j]);
+    }
+    if (TOGETHER && add) {
       float av[4];
       ar[j].get(av);
 #pragma unroll
