@@ -411,31 +411,44 @@ int dma_splits(long tiles, int ksteps) {
   return p2;
 }
 
-// What a product takes on one of the direct-to-LDS tilings below 256 x 256, in us: rounds of tiles over the chip, each
-// K steps long, and a split's second launch with its partial sums (8 bytes per output element and split, out of the
-// caches). The smaller tiles' rounds count whole (the last one's latency is not hidden), the others' in part (two or
-// three workgroups share a compute unit). Fitted to 512 .. 8192 rows, 512 .. 3072 columns over K = 512 .. 16384 in
-// all three layouts, within 15 % nearly everywhere.
-double dma_us(int variant, long m, long n, long batches, int ksteps, int splits, bool a_km, bool activation, long cus) {
+// What a product takes on one of the direct-to-LDS tilings below 256 x 256, in us: what a launch costs around its K
+// steps, the steps, the store pass by output elements, and a split's second launch with its partial sums (8 bytes per
+// element and split, out of the caches). A step takes `one` with at most one tile per compute unit and `more` for each
+// tile of the fullest unit beyond that: its tiles share the LDS, so each waits for less. (256 x 128 tiles, whose eight
+// waves start the next tile while others finish, go by the mean instead.) An output whose rows are not 16-byte aligned is
+// stored value by value, a tile's worth per round.
+// Fitted by least squares to 2500 timings: 256 .. 8192 rows, 333 .. 3072 columns, K = 512 .. 16384 split 1 to 16
+// ways, all layouts: 8 % rms. What it picks is 1 % behind the fastest on average (weight gradients of 1024 x 1024 over
+// 8192 / 16384 tokens: 34.1 / 55.9 -> 29.9 / 44.2 us, of 768 x 768 over 4096: 24.7 -> 16.0, against one step time for
+// every number of tiles on a unit and a larger tiling judged at one split only).
+double dma_us(int variant, long m, long n, long batches, int ksteps, int splits, bool a_km, bool activation, bool unaligned,
+              long cus) {
+  struct Cost {
+    double base, activation, unaligned, one[2], more[2];  // [k-contiguous A, k-major A]
+  };
+  static constexpr Cost kCosts[4] = {{3.5, 2.8, 7.5, {0.70, 0.64}, {0.86, 0.80}},    // 3: 256 x 128
+                                     {3.0, 1.5, 8.0, {0.51, 0.53}, {0.44, 0.39}},    // 6: 128 x 128
+                                     {3.4, 0.9, 2.2, {0.32, 0.35}, {0.245, 0.27}},   // 7: 128 x 64
+                                     {2.7, 0.7, 1.6, {0.20, 0.21}, {0.17, 0.18}}};   // 8: 64 x 64
+  const Cost& c = kCosts[variant == 3 ? 0 : variant - 5];
   int bm, bn;
   omx_gemm_dma_tile(variant, &bm, &bn);
   const long groups = ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batches * splits;
-  const double rounds = variant >= 7 || groups < cus ? static_cast<double>((groups + cus - 1) / cus)
-                                                     : static_cast<double>(groups) / static_cast<double>(cus);
-  // (a larger tile's store pass takes longer, an activation's more so; 64 columns of a k-major row are one cache line; 1024 x 1024
-  // over 8192 tokens unsplit: 34.9 us, 31.7 on 128 x 128 tiles with K split)
-  const double base = variant == 8 ? 3.0 : variant == 7 ? 3.5 : variant == 6 ? (activation ? 5.0 : 4.0) : activation ? 7.5 : 4.5;
-  const double step = variant == 8 ? (a_km ? 0.26 : 0.19) : variant == 7 ? 0.31 : variant == 6 ? 0.65 : 0.95;
-  return base + step * rounds * ((ksteps + splits - 1) / splits) +
-         (splits > 1 ? 6.0 + 1e-6 * static_cast<double>(m * n * splits) : 0.0);
+  const double fullest = variant == 3 ? static_cast<double>(groups) / static_cast<double>(cus)
+                                      : static_cast<double>((groups + cus - 1) / cus);
+  const double step = groups <= cus ? c.one[a_km] : std::max(c.one[a_km], c.more[a_km] * fullest);
+  const double out = 1e-6 * static_cast<double>(m) * static_cast<double>(n) * static_cast<double>(batches);
+  return c.base + (activation ? c.activation : 0.0) + (unaligned ? c.unaligned * std::max(1.0, fullest) : 0.0) +
+         step * ((ksteps + splits - 1) / splits) + 0.7 * out + (splits > 1 ? 5.8 + 0.17 * splits + 1.05 * out * splits : 0.0);
 }
 
-// The cheapest split of a product over tiling 6, 7 or 8, at most `limit` ways.
-int small_tile_splits(int variant, long m, long n, long batches, int ksteps, int limit, bool a_km, bool activation, long cus) {
+// The cheapest split of a product over such a tiling, at most `limit` ways.
+int cheapest_split(int variant, long m, long n, long batches, int ksteps, int limit, bool a_km, bool activation, bool unaligned,
+                   long cus) {
   int best = 1;
   for (int s = 2; s <= limit && ksteps / s >= 8; s *= 2)
-    if (dma_us(variant, m, n, batches, ksteps, s, a_km, activation, cus) <
-        dma_us(variant, m, n, batches, ksteps, best, a_km, activation, cus))
+    if (dma_us(variant, m, n, batches, ksteps, s, a_km, activation, unaligned, cus) <
+        dma_us(variant, m, n, batches, ksteps, best, a_km, activation, unaligned, cus))
       best = s;
   return best;
 }
@@ -517,7 +530,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
                     omx_gemm_thin_eligible(g, a_km, b_km);
   // Few rows (a decoder's linear layers): K shared between a workgroup's waves, no tile of 128 rows.
   const double skinny_us = operand_dtype == OMX_BF16 && !thin && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
-                               ? omx_gemm_skinny_us(ctx, g, a_km, b_km) : -1.0;
+                               ? omx_gemm_skinny_us(ctx, g, a_km, b_km, epi && epi->mode != OMX_EPI_NONE) : -1.0;
   bool skinny = skinny_us >= 0.0;
   // f32 outputs of less than a few rounds of 128 x 128 tiles.
   int frag32 = -1;
@@ -603,14 +616,14 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       }
       // A few hundred to a few thousand tokens, or a model some hundred wide, make less than a round or two of those
       // tiles. Two smaller ones in 64-column steps (whole cache lines of a k-contiguous row), where
-      // they take a tenth less than the choice above, or a fifth less than the few-row kernel, whose
+      // they take less than the choice above, or a fifth less than the few-row kernel, whose
       // workgroups have all of cold weights in flight at once:
       //   7  128 x 64, four waves, two workgroups per compute unit;
       //   8  64 x 64, four waves, three per compute unit.
       // A K step costs them 1.5 to 2 times the LDS traffic per product, so full rounds of the larger tiles stay there.
       // 3500 x 512 over K = 512 / 2048: 10.0 / 27.6 -> 5.8 / 14.4 us; 1024 x 3072 over 768 with GELU 17.3 -> 11.7;
       // 1024 x 768 over 768: 9.1 -> 5.1; six weight gradients of 512 x 512 over 3500: 54 -> 25. Scratch for a split
-      // stays within what the choice above would have taken.
+      // stays within what the choice above would have taken. That choice takes part at its own best split.
       if (dma_variant < 9) {
         const int ks = static_cast<int>(ksteps64);
         int bm = 128, bn = 128;
@@ -620,14 +633,18 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
         const int before = may_split && dma_variant >= 0 ? dma_splits(tiles, ks) : 1;
         const int limit = may_split && dma_variant < 0 ? static_cast<int>(std::min<long>((512 + tiles - 1) / tiles, ks / 8))
                                                        : before;
-        double best = skinny            ? 0.8 * skinny_us
-                      : dma_variant < 0 ? 1e30
-                                        : 0.9 * dma_us(dma_variant, g.M, g.N, g.batches, ks, before, a_km, !plain, cus);
+        auto splits_of = [&](int v) { return cheapest_split(v, g.M, g.N, g.batches, ks, limit, a_km, !plain, !g.c_vec, cus); };
+        auto us_of = [&](int v, int s) { return dma_us(v, g.M, g.N, g.batches, ks, s, a_km, !plain, !g.c_vec, cus); };
+        const int first = skinny ? -1 : dma_variant;
+        double best = skinny ? 0.8 * skinny_us : 1e30;
+        if (first >= 0) {
+          small_splits = splits_of(first);
+          best = us_of(first, small_splits);
+        }
         for (int v = 6; v <= 8; ++v) {
-          if (v == dma_variant) continue;
-          const int s = small_tile_splits(v, g.M, g.N, g.batches, ks, limit, a_km, !plain, cus);
-          const double us = dma_us(v, g.M, g.N, g.batches, ks, s, a_km, !plain, cus);
-          if (us < best) {
+          const int s = splits_of(v);
+          const double us = us_of(v, s);
+          if (v != first && us < best) {
             best = us;
             dma_variant = v;
             small_splits = s;

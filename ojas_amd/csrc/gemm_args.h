@@ -284,7 +284,7 @@ bool omx_gemm_thin_eligible(const GemmArgs& g, bool a_km, bool b_km);
 int32_t omx_gemm_thin_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km);
 
 // bf16 kernel for products of few rows or few outputs, both operands k-contiguous, K a multiple of 32.
-double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km);
+double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, bool activation);
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);
 
 // f32 kernel for small outputs: the tile it would take, or -1; the launch takes what the first returned.

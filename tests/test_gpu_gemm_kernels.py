@@ -114,6 +114,45 @@ def test_the_dispatcher_picks_a_tiling_within_a_tenth_of_the_best(be, layout, m,
     assert chosen <= 1.10 * fastest, (chosen, forced)
 
 
+@pytest.mark.parametrize("m,tokens,n", [(768, 4096, 768), (1024, 8192, 1024), (512, 16384, 512), (1024, 16384, 1024),
+                                        (2048, 16384, 512), (2048, 16384, 1024)])
+def test_long_weight_gradients_take_a_tiling_within_a_tenth_of_the_best(be, m, tokens, n):
+    """Weight gradients of one to four 128 x 128 tiles per eight compute units, where the tiling, its split and what shares
+    a unit weigh against each other: the choice against the tilings below 256 x 256 forced in turn, the small ones unsplit.
+    The kernels' own time, as the best of three runs of ten launches each."""
+    from ojas_amd.backend import BF16
+
+    print(f"gemm tiling choice, weight gradient {m}x{n} over {tokens}", flush=True)
+    a, b, c = be.empty((tokens * m,), BF16), be.empty((tokens * n,), BF16), be.empty((m, n))
+    for t, seed in ((a, 1), (b, 2)):
+        be._check(be._lib.omx_init_normal(be._ctx, be._p(t), C.c_int32(BF16), C.c_uint64(t.numel), C.c_uint64(seed),
+                                          C.c_float(0.05)))
+
+    def us(mode):
+        be.set_option("gemm_dma", mode)
+        best = float("inf")
+        for _ in range(3):
+            be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(1)))
+            for _ in range(10):
+                be._check(be._lib.omx_gemm(be._ctx, be._p(a), C.c_uint64(1), C.c_uint64(m), be._p(b), C.c_uint64(n), C.c_uint64(1),
+                                           C.c_int32(BF16), be._p(c), C.c_int32(0), C.c_uint64(m), C.c_uint64(tokens), C.c_uint64(n),
+                                           C.c_int32(0)))
+            ms = C.c_double()
+            be._check(be._lib.omx_profile_gemm_report(be._ctx, None, C.byref(ms), None))
+            be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(0)))
+            best = min(best, ms.value * 100)
+        return best
+
+    try:
+        us(1)  # clocks up
+        forced = {mode: us(mode) for mode in (3, 4, 7, 8)}
+        chosen = us(1)
+    finally:
+        be.set_option("gemm_dma", 1)
+    print("  us: chosen %.1f, forced %s" % (chosen, {mode: round(t, 1) for mode, t in forced.items()}), flush=True)
+    assert chosen <= 1.10 * min(forced.values()), (chosen, forced)
+
+
 def test_a_mostly_empty_last_round_is_cut_by_rows(be):
     """65 x 16 tiles of 256 x 256 are four rounds of the 256 compute units and 16 tiles more: the
     first 64 tile rows keep the tiling, the last goes to a launch of its own. Checked against the
