@@ -361,6 +361,25 @@ def test_small_tiles_end_a_reduction_inside_a_step(be, mode, tokens, m, n, pitch
     test_reductions_of_any_length_end_inside_a_step(be, mode, tokens, m, n, pitch)
 
 
+# More than one workgroup per compute unit of 256, where the small tiles keep three stages instead of five or six: 17 x 18 tiles
+# of 128 x 64, 33 x 18 of 64 x 64.
+@pytest.mark.parametrize("mode", [7, 8])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("m,k,n", [(2100, 64, 1100), (2100, 640, 1100)])
+def test_small_tiles_that_share_a_compute_unit(be, mode, layout, m, k, n):
+    test_small_direct_to_lds_tiles(be, mode, layout, m, k, n)
+
+
+@pytest.mark.parametrize("mode", [7, 8])
+def test_small_tiles_that_share_a_compute_unit_with_gelu(be, mode):
+    test_small_direct_to_lds_tiles_with_gelu(be, mode, 2100, 320, 1100)
+
+
+@pytest.mark.parametrize("mode", [7, 8])
+def test_small_tiles_that_share_a_compute_unit_end_a_reduction_inside_a_step(be, mode):
+    test_reductions_of_any_length_end_inside_a_step(be, mode, 333, 2100, 1104, 2104)
+
+
 @pytest.mark.parametrize("rows,kin,nout,layers", [(4096, 16, 512, 6), (4096, 384, 48, 5), (2048, 8, 256, 16)])
 def test_strided_batch_of_thin_weight_gradients_splits_the_reduction(be, rows, kin, nout, layers):
     """A batch of thin outputs over a long reduction (an adapter's rank x d gradients over the
