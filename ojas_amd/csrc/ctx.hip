@@ -295,6 +295,15 @@ int32_t omx_unsupported(omx_ctx* ctx, const char* op) {
 
 }  // extern "C"
 
+namespace {
+uint64_t workspace_size(uint64_t bytes) { return (bytes + (1ull << 20) - 1) & ~((1ull << 20) - 1); }
+}  // namespace
+
+bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot) {
+  const uint64_t held = ctx->workspace_bytes[slot];
+  return bytes <= held || ctx->budget_limit == 0 || ctx->budget_live - held + workspace_size(bytes) <= ctx->budget_limit;
+}
+
 int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot) {
   if (bytes <= ctx->workspace_bytes[slot]) {
     *out = ctx->workspace[slot];
@@ -313,7 +322,7 @@ int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot) {
     ctx->workspace[slot] = nullptr;
     ctx->workspace_bytes[slot] = 0;
   }
-  uint64_t rounded = (bytes + (1ull << 20) - 1) & ~((1ull << 20) - 1);
+  const uint64_t rounded = workspace_size(bytes);
   int32_t rc = omx_alloc(ctx, rounded, &ctx->workspace[slot]);
   if (rc != OMX_OK) return rc;
   ctx->workspace_bytes[slot] = rounded;

@@ -695,7 +695,8 @@ int32_t omx_cached_attention_forward(omx_ctx* ctx, const void* q, const void* k_
 
   // A prompt chunk: from 16 rows per KV head on, every tile of keys serves 16 rows and more, and the products go to
   // the matrix units (the kernels below read a key's row once per 4 or 8 query rows and take the sums on vector
-  // instructions). 4 x 12 heads, 256 new positions of 700: 186 -> 38 us per call.
+  // instructions). 4 x 12 heads, 256 new positions of 700: 186 -> 38 us per call. Where those rows make few workgroups over
+  // a long cache, the keys are split over more of them and the merge kernel adds the parts up.
   const bool bf16 = cache_dtype == OMX_BF16;
   const long step = static_cast<long>(kv_heads * head_dim);
   if (tq * (heads / kv_heads) >= 16 && tq * (heads / kv_heads) <= 0x7fffffffull && ctx->kv_attention_mode == 0 &&
@@ -721,7 +722,26 @@ int32_t omx_cached_attention_forward(omx_ctx* ctx, const void* q, const void* k_
     m.scale = 1.0f / std::sqrt(static_cast<float>(head_dim));
     m.fault = ctx->fault;
     m.tag = omx_tag(ctx, F_CACHED_ATTENTION);
-    return omx_sdpa32_forward(ctx, m, static_cast<int>(batch), static_cast<int>(head_dim), bf16);
+    // Few rows over a long cache: their keys are split over workgroups (without the scratch for it, one walks them all).
+    m.nparts = omx_sdpa32_key_parts(ctx, m, static_cast<int>(batch), static_cast<int>(head_dim), bf16);
+    const uint64_t bytes = rows_total * m.nparts * (head_dim + 2) * sizeof(float);
+    void* ws = nullptr;
+    if (m.nparts > 1 && (!omx_workspace_fits(ctx, bytes) || omx_workspace(ctx, bytes, &ws) != OMX_OK)) m.nparts = 1;
+    m.partial = m.nparts > 1 ? static_cast<float*>(ws) : nullptr;
+    const int32_t rc = omx_sdpa32_forward(ctx, m, static_cast<int>(batch), static_cast<int>(head_dim), bf16);
+    if (rc != OMX_OK || m.nparts == 1) return rc;
+    KvArgs merge{};
+    merge.partial = m.partial;
+    merge.nparts = m.nparts;
+    merge.out = m.out;
+    merge.dim = static_cast<int>(head_dim);
+    merge.fault = m.fault;
+    merge.tag = m.tag;
+    const long rows = static_cast<long>(rows_total);
+    omx_launch(ctx, (head_dim <= 64 ? &cached_attention_merge_kernel<1> : &cached_attention_merge_kernel<2>),
+               dim3(static_cast<unsigned>(rows)), dim3(64), 0, merge, rows);
+    OMX_LAUNCH_CHECK(ctx, "cached_attention_merge_kernel");
+    return OMX_OK;
   }
 
   KvArgs a;

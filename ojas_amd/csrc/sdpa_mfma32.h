@@ -16,6 +16,10 @@ struct Sdpa32Args {
   float *gq, *gk, *gv;
   float* delta;       // [batch, heads, tq]
   float* parts;       // set by the backward itself
+  // Forward over a cache with the keys split over workgroups: [batch, tq, heads][nparts][dim + 2], a part's unnormalised
+  // output, its maximum (natural logarithm) and its sum; null: the output itself.
+  float* partial;
+  int nparts;
   long q_b, q_h, q_t, k_b, k_h, k_t, o_b, o_h, o_t;
   int kv_heads, rep, tq, tk, q_pos0, slot0, capacity, window;
   float scale;
@@ -25,5 +29,7 @@ struct Sdpa32Args {
 
 // Head dims 16 / 32 / 64 / 128, 16-byte aligned tensors and strides, at most 65535 (batch, KV head) planes.
 bool omx_sdpa32_supports(uint64_t dim, uint64_t planes, std::initializer_list<const void*> ptrs, std::initializer_list<long> strides);
+// Into how many parts the forward over a cache had better split each row's keys (1: none).
+int omx_sdpa32_key_parts(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache);
 int32_t omx_sdpa32_forward(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache);
 int32_t omx_sdpa32_backward(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim);

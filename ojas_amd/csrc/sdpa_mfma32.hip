@@ -154,6 +154,20 @@ __device__ __forceinline__ bool at_store(float* row, const floatx4_a (&out)[AtDi
   return bad;
 }
 
+// Where part blockIdx.z of a row's result goes (Sdpa32Args::partial).
+__device__ __forceinline__ float* at_partial(const Sdpa32Args& a, int dim, int b, int kvh, int query, int head) {
+  const long row = (static_cast<long>(b) * a.tq + query) * a.kv_heads * a.rep + static_cast<long>(kvh) * a.rep + head;
+  return a.partial + (row * a.nparts + blockIdx.z) * (dim + 2);
+}
+// This workgroup's share of the tiles first .. last: all of them, or part blockIdx.z (which may be empty).
+__device__ __forceinline__ void at_key_part(const Sdpa32Args& a, int* first, int* last) {
+  if (a.nparts > 1) {
+    const int each = (*last - *first + a.nparts) / a.nparts;
+    *first += static_cast<int>(blockIdx.z) * each;
+    *last = min(*last, *first + each - 1);
+  }
+}
+
 struct AtRow {
   int query, head;  // head within the group
 };
@@ -197,19 +211,21 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   const int low = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
   const int first_pos = a.q_pos0 + at_unpack(r0, a.rep).query;
   const int last_pos = a.q_pos0 + at_unpack(min(r0 + BQ, rows) - 1, a.rep).query;
-  const int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / AT_ROWS, t_last = last_pos / AT_ROWS;
+  int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / AT_ROWS, t_last = last_pos / AT_ROWS;
+  at_key_part(a, &t_first, &t_last);
   const TK* kb = static_cast<const TK*>(a.k) + b * a.k_b + kvh * a.k_h;
   const TK* vb = static_cast<const TK*>(a.v) + b * a.k_b + kvh * a.k_h;
   AtTile<D, TK> kn, vn;
   auto fetch = [&](int t) {
-    auto slot_at = [&](int row) {
+    auto row_of = [&](const TK* base, int row) {
       const int key = t * AT_ROWS + row;
-      int slot = a.slot0 + key;  // a ring wraps at most once over the keys that are read
-      slot = slot >= a.capacity ? slot - a.capacity : slot;
-      return key < a.tk ? slot : -1;
+      // A ring wraps at most once over the keys that are read (slot0 + key can pass 2^31).
+      unsigned int slot = static_cast<unsigned int>(a.slot0) + key;
+      slot = slot >= static_cast<unsigned int>(a.capacity) ? slot - a.capacity : slot;
+      return key < a.tk ? base + static_cast<long>(slot) * a.k_t : nullptr;
     };
-    kn.fetch([&](int row) { const int s = slot_at(row); return s < 0 ? nullptr : kb + static_cast<long>(s) * a.k_t; });
-    vn.fetch([&](int row) { const int s = slot_at(row); return s < 0 ? nullptr : vb + static_cast<long>(s) * a.k_t; });
+    kn.fetch([&](int row) { return row_of(kb, row); });
+    vn.fetch([&](int row) { return row_of(vb, row); });
   };
   const float scale2 = a.scale * AT_LOG2E;
   floatx4_a o[X::S];
@@ -217,7 +233,7 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   for (int m = 0; m < X::S; ++m) o[m] = at_zero();
   float mx = -INFINITY, sum = 0.0f;  // in the exp2 domain; `sum` over this lane's keys only
   bool bad = false;
-  fetch(t_first);
+  if (t_first <= t_last) fetch(t_first);
   for (int t = t_first; t <= t_last; ++t) {
     __syncthreads();  // the previous tile has been read
     kn.store(kt);
@@ -262,11 +278,22 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   sum = at_row_sum(sum);
   float* out = a.out + b * a.o_b + (static_cast<long>(kvh) * a.rep + at.head) * a.o_h + static_cast<long>(at.query) * a.o_t;
   float* lse = a.lse ? a.lse + (static_cast<long>(b) * a.kv_heads * a.rep + static_cast<long>(kvh) * a.rep + at.head) * a.tq + at.query : nullptr;
+  // A part's maximum and sum, by one lane of the row.
+  auto store_part = [&](float top, float total, float* row) {
+    row[D] = top * AT_LN2;  // (minus infinity where the row saw none of the part's keys)
+    row[D + 1] = total;
+  };
   if constexpr (KW == 1) {
     if (r < rows) {
-      bad |= !(dev_finite(sum) && sum > 0.0f);
-      bad |= at_store<D, 4>(out, o, 1.0f / sum, g, 0);
-      if (lse && g == 0) *lse = mx * AT_LN2 + logf(sum);
+      if (a.nparts > 1) {
+        float* row = at_partial(a, D, b, kvh, at.query, at.head);
+        bad |= at_store<D, 4>(row, o, 1.0f, g, 0);
+        if (g == 0) store_part(mx, sum, row);
+      } else {
+        bad |= !(dev_finite(sum) && sum > 0.0f);
+        bad |= at_store<D, 4>(out, o, 1.0f / sum, g, 0);
+        if (lse && g == 0) *lse = mx * AT_LN2 + logf(sum);
+      }
     }
   } else {
     // The four waves' shares of the same rows: every wave adds up one register of each block.
@@ -299,9 +326,15 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
       o[m] = floatx4_a{x, x, x, x};
     }
     if (r < rows) {
-      bad |= !(dev_finite(total) && total > 0.0f);
-      bad |= at_store<D, 1>(out, o, 1.0f / total, g, kw);
-      if (lse && g == 0 && kw == 0) *lse = all * AT_LN2 + logf(total);
+      if (a.nparts > 1) {
+        float* row = at_partial(a, D, b, kvh, at.query, at.head);
+        bad |= at_store<D, 1>(row, o, 1.0f, g, kw);
+        if (g == 0 && kw == 0) store_part(all, total, row);
+      } else {
+        bad |= !(dev_finite(total) && total > 0.0f);
+        bad |= at_store<D, 1>(out, o, 1.0f / total, g, kw);
+        if (lse && g == 0 && kw == 0) *lse = all * AT_LN2 + logf(total);
+      }
     }
   }
   if (bad) dev_raise_fault(a.fault, a.tag);
@@ -357,8 +390,8 @@ struct AtPrompt {
   static constexpr int PIECES = KEYS * D / 8 / 64;
 };
 
-// (three workgroups per compute unit with one block of rows: 168 registers)
-template <int D, int MB>
+// (three workgroups per compute unit with one block of rows: 168 registers, none to spare for the parts of split keys)
+template <int D, int MB, bool SPLIT>
 __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_prompt_kernel(Sdpa32Args a) {
   using X = AtPrompt<D>;
   __shared__ __align__(16) char lds[4 * X::KEYS * X::PITCH];
@@ -386,15 +419,17 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
   }
   const int first_pos = a.q_pos0 + at_unpack(r0, a.rep).query;
   const int last_pos = a.q_pos0 + at_unpack(min(r0 + 16 * MB, rows) - 1, a.rep).query;
-  const int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / X::KEYS, t_last = last_pos / X::KEYS;
+  int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / X::KEYS, t_last = last_pos / X::KEYS;
+  if constexpr (SPLIT) at_key_part(a, &t_first, &t_last);
   const unsigned short* kb = static_cast<const unsigned short*>(a.k) + b * a.k_b + kvh * a.k_h;
   const unsigned short* vb = static_cast<const unsigned short*>(a.v) + b * a.k_b + kvh * a.k_h;
   char* region = lds + wave * (X::KEYS * X::PITCH);
 
   u32x4_a kn[X::NB][X::KS], vn[X::PIECES];
   auto slot_at = [&](int key) {
-    int slot = a.slot0 + key;  // a ring wraps at most once over the keys that are read
-    return static_cast<long>(slot >= a.capacity ? slot - a.capacity : slot) * a.k_t;
+    // A ring wraps at most once over the keys that are read (slot0 + key can pass 2^31).
+    const unsigned int slot = static_cast<unsigned int>(a.slot0) + key, capacity = a.capacity;
+    return static_cast<long>(slot >= capacity ? slot - capacity : slot) * a.k_t;
   };
   auto fetch = [&](int t) {  // keys past the last one are rows of zeros
 #pragma unroll
@@ -524,9 +559,17 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
       total = fmaf(weight[w], stat[w * 32 + 16 + i], total);
     }
     if (r0 + m * 16 + i < rows) {
-      bad |= !(dev_finite(total) && total > 0.0f);
-      const float f = 1.0f / total;
-      float* out = a.out + b * a.o_b + (static_cast<long>(kvh) * a.rep + at[m].head) * a.o_h + static_cast<long>(at[m].query) * a.o_t;
+      if constexpr (SPLIT) {
+        if (wave == 0 && g == 0) {
+          float* row = at_partial(a, D, b, kvh, at[m].query, at[m].head);
+          row[D] = all * AT_LN2;
+          row[D + 1] = total;
+        }
+      } else {
+        bad |= !(dev_finite(total) && total > 0.0f);
+      }
+      const float f = SPLIT ? 1.0f : 1.0f / total;
+      float* out = SPLIT ? at_partial(a, D, b, kvh, at[m].query, at[m].head) : a.out + b * a.o_b + (static_cast<long>(kvh) * a.rep + at[m].head) * a.o_h + static_cast<long>(at[m].query) * a.o_t;
 #pragma unroll
       for (int d0 = 0; d0 < X::DB; d0 += 4) {
         float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -543,7 +586,13 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
           x[v] *= f;
           bad |= !dev_finite(x[v]);
         }
-        *reinterpret_cast<float4*>(out + (d0 + wave) * 16 + 4 * g) = make_float4(x[0], x[1], x[2], x[3]);
+        float* to = out + (d0 + wave) * 16 + 4 * g;
+        if constexpr (SPLIT) {  // (a part's rows are 8-byte aligned)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) to[v] = x[v];
+        } else {
+          *reinterpret_cast<float4*>(to) = make_float4(x[0], x[1], x[2], x[3]);
+        }
       }
     }
   }
@@ -801,26 +850,29 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_parts_kernel(Sdpa32Args a, 
 // without a workgroup (8 x 4 heads x 256: forward 17.5 -> 12.9 us, backward 46 -> 34; 4 heads x 2048: 114 -> 69, 241 -> 190).
 bool at_narrow(omx_ctx* ctx, long planes, long rows) { return planes * ((rows + 63) / 64) < ctx->cu_count; }
 
+// Rows per workgroup of the forward.
+long forward_rows(omx_ctx* ctx, int dim, long planes, long rows, bool bf16_cache) {
+  if (dim >= 64 && bf16_cache)  // Twice the rows on a key's way only where half as many workgroups still fill the chip.
+    return dim == 64 && (rows + 31) / 32 * planes >= 4l * (ctx->cu_count > 0 ? ctx->cu_count : 256) ? 32 : 16;
+  return at_narrow(ctx, planes, rows) ? 16 : 64;
+}
+
 template <int D>
 int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) {
-  const long rows = static_cast<long>(a.tq) * a.rep;
+  const long rows = static_cast<long>(a.tq) * a.rep, per = forward_rows(ctx, D, planes, rows, bf16_cache);
+  const dim3 grid(static_cast<unsigned>((rows + per - 1) / per), planes, static_cast<unsigned>(std::max(1, a.nparts)));
   if constexpr (D >= 64) {
     if (bf16_cache) {  // (attention over a cache has no lse)
-      // Twice the rows on a key's way only where half as many workgroups still fill the chip.
-      const bool two = D == 64 && (rows + 31) / 32 * planes >= 4l * (ctx->cu_count > 0 ? ctx->cu_count : 256);
-      const long per = two ? 32 : 16;
-      dim3 blocks(static_cast<unsigned>((rows + per - 1) / per), planes);
+      const bool two = per == 32, split = a.nparts > 1;  // (two: four workgroups per compute unit and more, never split)
       if constexpr (D == 64) {
-        if (two) omx_launch(ctx, (sdpa_prompt_kernel<D, 2>), blocks, dim3(AT_THREADS), 0, a);
+        if (two) omx_launch(ctx, (sdpa_prompt_kernel<D, 2, false>), grid, dim3(AT_THREADS), 0, a);
       }
-      if (!two) omx_launch(ctx, (sdpa_prompt_kernel<D, 1>), blocks, dim3(AT_THREADS), 0, a);
+      if (!two) omx_launch(ctx, (split ? &sdpa_prompt_kernel<D, 1, true> : &sdpa_prompt_kernel<D, 1, false>), grid, dim3(AT_THREADS), 0, a);
       OMX_LAUNCH_CHECK(ctx, "sdpa_prompt_kernel");
       return OMX_OK;
     }
   }
-  const bool narrow = at_narrow(ctx, planes, rows);
-  const long bq = narrow ? 16 : 64;
-  dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
+  const bool narrow = per == 16;
   using Cache = std::conditional_t<(D < 64), unsigned short, float>;  // bf16 caches of wider heads are gone by now
   auto launch_bf16 = [&](auto kernel) { omx_launch(ctx, kernel, grid, dim3(AT_THREADS), 0, a); };
   if (narrow) {
@@ -880,6 +932,33 @@ bool omx_sdpa32_supports(uint64_t dim, uint64_t planes, std::initializer_list<co
   for (long s : strides)
     if (s % 4 != 0) return false;
   return true;
+}
+
+// A workgroup's chain of steps (each one set of keys for all of its rows) in us, slower by what shares its compute unit (the
+// bf16 form is bound by vector instructions, two workgroups of the f32 one take 1.36 times as long as one), against a second
+// launch that adds the parts up, 0.55 us for each. 16 heads over one KV head x 64, one new token, 8192 positions, one
+// workgroup without parts: 68 -> 20 us over a bf16 cache, 204 -> 28 over an f32 one; 12 heads x 16 new tokens 70 -> 20 and
+// 206 -> 30; 1024 positions 12.5 -> 11 and 28 -> 14. (The kernels for few rows: 85, 85; 82, 88; 24, 24.)
+int omx_sdpa32_key_parts(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache) {
+  const long rows = static_cast<long>(a.tq) * a.rep, planes = static_cast<long>(batch) * a.kv_heads;
+  const long per = forward_rows(ctx, dim, planes, rows, bf16_cache), blocks = (rows + per - 1) / per * planes;
+  const bool prompt = dim >= 64 && bf16_cache;
+  const long keys = prompt ? 4 * (4096 / dim) : AT_ROWS;
+  const double step = prompt ? (dim == 64 ? 2.0 : 1.45) : 0.5 + 0.0175 * dim;
+  const long steps = (a.tk + keys - 1) / keys, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const long most = std::min(std::min(2 * cus / blocks, steps), 64l);
+  long best = 1;
+  double least = 0.0;
+  for (long p = 1; p <= std::max(1l, most); ++p) {
+    const long shared = (blocks * p + cus - 1) / cus;  // on the fullest compute unit
+    const double slower = shared == 1 ? 1.0 : prompt ? static_cast<double>(shared) : 0.68 * static_cast<double>(shared);
+    const double us = static_cast<double>((steps + p - 1) / p) * step * slower + (p > 1 ? 3.0 + 0.55 * static_cast<double>(p) : 0.0);
+    if (p == 1 || us < least) {
+      best = p;
+      least = us;
+    }
+  }
+  return static_cast<int>(best);
 }
 
 int32_t omx_sdpa32_forward(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache) {
