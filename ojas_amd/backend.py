@@ -581,6 +581,13 @@ class MiBackend(_native.Methods):
 
     def muon_ns5_step_batched(self, params, grads, momenta, config: MuonNs5Config, params_bf16=None):
         """`muon_ns5_step` on several tensors of one shape in one set of launches (in place)."""
+        self._muon_list(_native.omx_muon_ns5_step_batched, params, grads, momenta, config, params_bf16)
+
+    def muon_ns5_step_list(self, params, grads, momenta, config: MuonNs5Config, params_bf16=None):
+        """The same within 256 MiB of scratch and whatever less the budget has room for."""
+        self._muon_list(_native.omx_muon_ns5_step_list, params, grads, momenta, config, params_bf16)
+
+    def _muon_list(self, entry, params, grads, momenta, config, params_bf16):
         n = len(params)
         rows, cols = params[0].shape
         if any(p.shape != (rows, cols) for p in params) or len(grads) != n or len(momenta) != n:
@@ -588,8 +595,7 @@ class MiBackend(_native.Methods):
         table = lambda ts: (C.c_void_p * n)(*[t.ptr for t in ts])
         mirrors = (C.c_void_p * n)(*[(t.ptr if t is not None else None) for t in params_bf16]) if params_bf16 else None
         tables = [table(ts) for ts in (params, grads, momenta)] + ([mirrors] if mirrors is not None else [])
-        _native.omx_muon_ns5_step_batched(self._context, *([C.addressof(t) for t in tables] + [None])[:4], n, rows, cols,
-                                          C.addressof(config))
+        entry(self._context, *([C.addressof(t) for t in tables] + [None])[:4], n, rows, cols, C.addressof(config))
 
     def clip_grad_norm(self, grads: Sequence[DeviceTensor], max_norm: float) -> float:
         ptrs, lens = self._pointers(grads), self._lengths(grads)

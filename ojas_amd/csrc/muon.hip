@@ -318,18 +318,31 @@ int32_t muon_scalars(omx_ctx* ctx, const char* op, const omx_muon_config* c, uin
   return OMX_OK;
 }
 
+// `bounded`: as many tensors at a time as MU_SCRATCH holds and the budget has room for, one at least.
+constexpr uint64_t MU_SCRATCH = 256ull << 20;
 int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void* const* grads, void* const* momenta,
-                   void* const* params_bf16, uint64_t count, uint64_t rows, uint64_t cols, const omx_muon_config* c) {
+                   void* const* params_bf16, uint64_t count, uint64_t rows, uint64_t cols, const omx_muon_config* c,
+                   bool bounded) {
   MuonScalars s;
   int32_t rc = muon_scalars(ctx, op, c, rows, cols, &s);
   if (rc != OMX_OK) return rc;
   for (uint64_t i = 0; i < count; ++i)
     if (!params[i] || !grads[i] || !momenta[i]) return omx_fail(ctx, OMX_PLACEMENT, "%s: null pointer", op);
   const MuonLayout L = muon_layout(rows, cols);
-  for (uint64_t first = 0; first < count; first += MU_MAX_BATCH) {
-    const unsigned n = static_cast<unsigned>(std::min<uint64_t>(MU_MAX_BATCH, count - first));
+  uint64_t most = MU_MAX_BATCH;
+  if (bounded) {
+    most = std::max<uint64_t>(1, std::min<uint64_t>(most, MU_SCRATCH / L.total));
+    most = std::min(most, count);
+    while (most > 1 && !omx_workspace_fits(ctx, L.total * most)) --most;
+  }
+  for (uint64_t first = 0; first < count;) {
+    unsigned n = static_cast<unsigned>(std::min<uint64_t>(most, count - first));
     void* ws = nullptr;
     rc = omx_workspace(ctx, L.total * n, &ws);
+    if (rc == OMX_CAPACITY_EXCEEDED && bounded && n > 1) {  // (no memory left on the device)
+      most = (n + 1) / 2;
+      continue;
+    }
     if (rc != OMX_OK) return rc;
     MuonTensors t{};
     for (unsigned i = 0; i < n; ++i) {
@@ -342,6 +355,7 @@ int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void
     rc = s.bf16 ? run_muon<unsigned short>(ctx, t, n, rows, cols, s, static_cast<char*>(ws), L, tag)
                 : run_muon<float>(ctx, t, n, rows, cols, s, static_cast<char*>(ws), L, tag);
     if (rc != OMX_OK) return rc;
+    first += n;
   }
   return OMX_OK;
 }
@@ -362,7 +376,7 @@ int32_t omx_muon_ns5_step(omx_ctx* ctx, void* param, const void* grad, void* mom
   if (!param || !grad || !momentum || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null pointer", op);
   void* mirrors[1] = {param_bf16};
   const void* grads[1] = {grad};
-  return muon_batch(ctx, op, &param, grads, &momentum, param_bf16 ? mirrors : nullptr, 1, rows, cols, c);
+  return muon_batch(ctx, op, &param, grads, &momentum, param_bf16 ? mirrors : nullptr, 1, rows, cols, c, false);
 }
 
 int32_t omx_muon_ns5_step_batched(omx_ctx* ctx, void* const* params, const void* const* grads, void* const* momenta,
@@ -372,7 +386,17 @@ int32_t omx_muon_ns5_step_batched(omx_ctx* ctx, void* const* params, const void*
   const char* op = "muon_ns5_step";
   if (!params || !grads || !momenta || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null pointer", op);
   if (count == 0) return omx_fail(ctx, OMX_SHAPE, "%s: no tensors", op);
-  return muon_batch(ctx, op, params, grads, momenta, params_bf16, count, rows, cols, c);
+  return muon_batch(ctx, op, params, grads, momenta, params_bf16, count, rows, cols, c, false);
+}
+
+int32_t omx_muon_ns5_step_list(omx_ctx* ctx, void* const* params, const void* const* grads, void* const* momenta,
+                               void* const* params_bf16, uint64_t count, uint64_t rows, uint64_t cols,
+                               const omx_muon_config* c) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "muon_ns5_step";
+  if (!params || !grads || !momenta || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null pointer", op);
+  if (count == 0) return omx_fail(ctx, OMX_SHAPE, "%s: no tensors", op);
+  return muon_batch(ctx, op, params, grads, momenta, params_bf16, count, rows, cols, c, true);
 }
 
 }  // extern "C"

@@ -279,8 +279,8 @@ class NanolabTrainer:
         # model's 32 matrices took 990 launches and its 25 vectors 75, most of the step's time.
         cfg = MuonNs5Config(self.matrix_lr * lr_multiplier, MUON_MOMENTUM, MUON_WEIGHT_DECAY, 1, int(self.ns5_bf16))
         for names in self.muon_groups:
-            be.muon_ns5_step_batched([self.params[n] for n in names], [acc[n] for n in names],
-                                     [self.state[n][0] for n in names], cfg)
+            be.muon_ns5_step_list([self.params[n] for n in names], [acc[n] for n in names],
+                                  [self.state[n][0] for n in names], cfg)
         cfg = AdamWConfig.nanolab(self.adam_lr * lr_multiplier, ADAM_HYBRID_WEIGHT_DECAY)
         be.adamw_step_batched([self.params[n] for n in self.adam], [acc[n] for n in self.adam],
                               [self.state[n][0] for n in self.adam], [self.state[n][1] for n in self.adam], self.step, cfg)

@@ -173,3 +173,47 @@ def test_bf16_iteration_sums_in_the_store_pass_carry_the_separate_kernels_bits(b
     for a, b in zip(got[1], got[0]):
         assert np.array_equal(a, b)
     assert any(np.any(a != p) for a, p in zip(got[1][:count], ps))
+
+
+@pytest.mark.parametrize("rows,cols,count,room,bf16", [(256, 256, 5, 2, 0), (96, 512, 7, 1, 1), (512, 96, 70, 64, 0)])
+def test_list_step_takes_the_scratch_there_is(be, rows, cols, count, room, bf16):
+    """`muon_ns5_step_list` with room for the scratch of `room` matrices: as many at a time, each held to the oracle."""
+    from ojas_amd.backend import CAPACITY_EXCEEDED, MiBackend, MuonNs5Config, OjasError
+
+    print(f"muon list {count} x {rows}x{cols}, room for {room}", flush=True)
+    r = np.random.default_rng(rows + count)
+    ps, gs, ms = ([r.standard_normal((rows, cols)).astype(np.float32) * s for _ in range(count)] for s in (0.1, 0.05, 0.01))
+    cfg = MuonNs5Config(0.02, 0.95, 0.1, 1, bf16)
+    each = int(be._lib.omx_muon_scratch_bytes(rows, cols))
+    rounded = (each * room + (1 << 20) - 1) >> 20 << 20
+    small = MiBackend(0, budget_bytes=3 * count * rows * cols * 4 + rounded)
+    dp, dg, dm = [small.upload(x) for x in ps], [small.upload(x) for x in gs], [small.upload(x) for x in ms]
+    if room < min(count, 64):
+        with pytest.raises(OjasError) as e:  # all of them at once do not fit
+            small.muon_ns5_step_batched(dp, dg, dm, cfg)
+        assert e.value.code == CAPACITY_EXCEEDED
+    small.muon_ns5_step_list(dp, dg, dm, cfg)
+    decay = np.float32(1.0 - 0.02 * 0.1)
+    for i in sorted({0, room - 1, room % count, count - 1}):
+        op, om = orc.muon_ns5_step(ps[i], gs[i], ms[i], lr=0.02, momentum=0.95, weight_decay=0.1, nesterov=True, bf16=bool(bf16))
+        assert np.array_equal(small.download(dm[i]), om), i
+        upd_gpu, upd_cpu = small.download(dp[i]) - ps[i] * decay, op - ps[i] * decay
+        assert np.max(np.abs(upd_gpu - upd_cpu)) <= (5e-2 if bf16 else 2e-3) * np.max(np.abs(upd_cpu)), i
+    small.close()
+
+
+def test_a_model_of_many_matrices_steps_within_its_budget():
+    """84 matrices of 512 x 512: 64 of them at once are 403 MB of scratch, one is 6.3."""
+    from ojas_amd.backend import MiBackend
+    from ojas_amd.nanolab import NanolabSpec, NanolabTrainer
+
+    print("muon: 84 matrices under a budget", flush=True)
+    be = MiBackend(0, budget_bytes=480 << 20)
+    spec = NanolabSpec(n_layer=12, n_embd=512, n_head=8, n_kv_head=8, head_dim=64, hidden=512, vocab=256, window=None, max_seq=16)
+    r = np.random.default_rng(2)
+    host = {n: (r.standard_normal(s) * 0.02 if len(s) == 2 else np.ones(s)).astype(np.float32) for n, s in spec.param_shapes().items()}
+    tr = NanolabTrainer(be, spec, host)
+    ids = r.integers(0, 256, (1, 16)).astype(np.uint32)
+    assert np.isfinite(tr.run([(ids, ids)], 0.1).loss)
+    del tr
+    be.close()
