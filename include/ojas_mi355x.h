@@ -424,8 +424,9 @@ int32_t omx_muon_ns5_step(omx_ctx* ctx, void* param_f32, const void* grad_f32, v
 int32_t omx_muon_ns5_step_batched(omx_ctx* ctx, void* const* params_f32, const void* const* grads_f32,
                                   void* const* momenta_f32, void* const* params_bf16, uint64_t count,
                                   uint64_t rows, uint64_t cols, const omx_muon_config* config);
-/* omx_muon_ns5_step_batched for a list of any length under any budget: its scratch is 256 MiB at most, as much of
- * that as the budget has room for, and omx_muon_ns5_step's at least. */
+/* omx_muon_ns5_step on each tensor of a list of one shape, in as few sets of launches as its scratch allows: 256 MiB at
+ * most, as much of that as the budget has room for, and omx_muon_ns5_step's at least. Each tensor is all-or-nothing by
+ * itself. */
 int32_t omx_muon_ns5_step_list(omx_ctx* ctx, void* const* params_f32, const void* const* grads_f32,
                                void* const* momenta_f32, void* const* params_bf16, uint64_t count,
                                uint64_t rows, uint64_t cols, const omx_muon_config* config);

@@ -584,7 +584,8 @@ class MiBackend(_native.Methods):
         self._muon_list(_native.omx_muon_ns5_step_batched, params, grads, momenta, config, params_bf16)
 
     def muon_ns5_step_list(self, params, grads, momenta, config: MuonNs5Config, params_bf16=None):
-        """The same within 256 MiB of scratch and whatever less the budget has room for."""
+        """The same, each tensor all-or-nothing by itself, within 256 MiB of scratch and whatever less the budget has
+        room for."""
         self._muon_list(_native.omx_muon_ns5_step_list, params, grads, momenta, config, params_bf16)
 
     def _muon_list(self, entry, params, grads, momenta, config, params_bf16):

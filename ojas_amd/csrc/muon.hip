@@ -13,7 +13,7 @@
 // the iterate then lives in bf16 storage and the three products run on the
 // bf16 MFMA lane, whose bf16 output store is exactly that rounding.
 //
-// The step is all-or-nothing: a refuse flag raised by any non-finite
+// The step is all-or-nothing, for the batch or (the list form) for each matrix: a refuse flag raised by any non-finite
 // intermediate keeps the final pass from writing the parameter or the momentum.
 #include <algorithm>
 #include <cmath>
@@ -53,7 +53,12 @@ struct MuonWork {
   char* ws;
   uint64_t stride;  // bytes between consecutive matrices' blocks
   MuonLayout L;
-  unsigned int* refuse;  // one flag for the whole launch
+  // The flag that keeps the final pass from writing: one for the launch (refuse_stride 0), or one for each matrix.
+  unsigned int* refuse;
+  uint64_t refuse_stride;
+  __device__ __forceinline__ unsigned int* flag() const {
+    return reinterpret_cast<unsigned int*>(reinterpret_cast<char*>(refuse) + blockIdx.y * refuse_stride);
+  }
   template <typename T>
   __device__ __forceinline__ T* at(uint64_t offset) const {
     return reinterpret_cast<T*>(ws + blockIdx.y * stride + offset);
@@ -90,9 +95,13 @@ __global__ __launch_bounds__(MU_THREADS) void muon_momentum_kernel(MuonTensors t
   }
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
   if (bad) {
-    atomicOr(w.refuse, 1u);
+    atomicOr(w.flag(), 1u);
     dev_raise_fault(fault, tag);
   }
+}
+
+__global__ void muon_clear_flags_kernel(MuonWork w) {
+  if (threadIdx.x == 0) *w.flag() = 0u;
 }
 
 // One block per matrix (blockIdx.y): the norm and the quotient's denominator.
@@ -114,7 +123,7 @@ __global__ __launch_bounds__(1024) void muon_norm_kernel(MuonWork w, size_t coun
     float denom = bf16 ? dev_round_bf16(dev_round_bf16(norm) + eps) : norm + eps;
     *w.at<float>(w.L.scalars + 16) = denom;
     if (!(dev_finite(denom) && denom != 0.0f)) {
-      atomicOr(w.refuse, 1u);
+      atomicOr(w.flag(), 1u);
       dev_raise_fault(fault, tag);
     }
   }
@@ -161,7 +170,7 @@ __global__ void muon_combine_x_kernel(MuonWork w, uint64_t x_off, uint64_t bx_of
     dev_store<TX>(bx, i, r);
   }
   if (bad) {
-    atomicOr(w.refuse, 1u);
+    atomicOr(w.flag(), 1u);
     dev_raise_fault(fault, tag);
   }
 }
@@ -178,14 +187,14 @@ __global__ void muon_check_update_kernel(MuonTensors t, MuonWork w, uint64_t x_o
     bad |= !dev_finite(fmaf(s.alpha, dev_load<TX>(x, i), base));
   }
   if (bad) {
-    atomicOr(w.refuse, 1u);
+    atomicOr(w.flag(), 1u);
     dev_raise_fault(fault, tag);
   }
 }
 
 template <typename TX>
 __global__ void muon_apply_kernel(MuonTensors t, MuonWork w, uint64_t x_off, size_t n, MuonScalars s) {
-  if (*w.refuse) return;
+  if (*w.flag()) return;
   float* __restrict__ p = t.p[blockIdx.y];
   float* __restrict__ m = t.m[blockIdx.y];
   unsigned short* __restrict__ p_bf16 = t.p16[blockIdx.y];
@@ -229,7 +238,7 @@ MuonLayout muon_layout(uint64_t rows, uint64_t cols) {
 // `count` (<= MU_MAX_BATCH) matrices of one shape; ws holds count blocks of L.total bytes.
 template <typename TX>
 int32_t run_muon(omx_ctx* ctx, const MuonTensors& t, unsigned count, uint64_t rows, uint64_t cols, MuonScalars s,
-                 char* ws, const MuonLayout& L, unsigned long long tag) {
+                 char* ws, const MuonLayout& L, bool each, unsigned long long tag) {
   const uint64_t len = rows * cols;
   const int32_t XD = sizeof(TX) == 2 ? OMX_BF16 : OMX_F32;
   MuonWork w;
@@ -237,8 +246,10 @@ int32_t run_muon(omx_ctx* ctx, const MuonTensors& t, unsigned count, uint64_t ro
   w.stride = L.total;
   w.L = L;
   w.refuse = reinterpret_cast<unsigned int*>(ws + L.scalars);
-  int32_t rc = omx_fill_zero(ctx, w.refuse, 4);
-  if (rc != OMX_OK) return rc;
+  w.refuse_stride = each ? L.total : 0;
+  omx_launch(ctx, muon_clear_flags_kernel, dim3(1, each ? count : 1), dim3(64), 0, w);
+  OMX_LAUNCH_CHECK(ctx, "muon_clear_flags_kernel");
+  int32_t rc = OMX_OK;
   uint64_t x_off = L.x, xn_off = L.xn;
   const unsigned nb = static_cast<unsigned>((len + MU_BLOCK - 1) / MU_BLOCK);
   const dim3 block(MU_THREADS), over_len(mu_grid(len), count);
@@ -318,11 +329,12 @@ int32_t muon_scalars(omx_ctx* ctx, const char* op, const omx_muon_config* c, uin
   return OMX_OK;
 }
 
-// `bounded`: as many tensors at a time as MU_SCRATCH holds and the budget has room for, one at least.
+// `list`: each tensor all-or-nothing by itself, and as many at a time as MU_SCRATCH holds and the budget has room for, one
+// at least.
 constexpr uint64_t MU_SCRATCH = 256ull << 20;
 int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void* const* grads, void* const* momenta,
                    void* const* params_bf16, uint64_t count, uint64_t rows, uint64_t cols, const omx_muon_config* c,
-                   bool bounded) {
+                   bool list) {
   MuonScalars s;
   int32_t rc = muon_scalars(ctx, op, c, rows, cols, &s);
   if (rc != OMX_OK) return rc;
@@ -330,7 +342,7 @@ int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void
     if (!params[i] || !grads[i] || !momenta[i]) return omx_fail(ctx, OMX_PLACEMENT, "%s: null pointer", op);
   const MuonLayout L = muon_layout(rows, cols);
   uint64_t most = MU_MAX_BATCH;
-  if (bounded) {
+  if (list) {
     most = std::max<uint64_t>(1, std::min<uint64_t>(most, MU_SCRATCH / L.total));
     most = std::min(most, count);
     while (most > 1 && !omx_workspace_fits(ctx, L.total * most)) --most;
@@ -339,7 +351,7 @@ int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void
     unsigned n = static_cast<unsigned>(std::min<uint64_t>(most, count - first));
     void* ws = nullptr;
     rc = omx_workspace(ctx, L.total * n, &ws);
-    if (rc == OMX_CAPACITY_EXCEEDED && bounded && n > 1) {  // (no memory left on the device)
+    if (rc == OMX_CAPACITY_EXCEEDED && list && n > 1) {  // (no memory left on the device)
       most = (n + 1) / 2;
       continue;
     }
@@ -352,8 +364,8 @@ int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void
       t.p16[i] = params_bf16 ? static_cast<unsigned short*>(params_bf16[first + i]) : nullptr;
     }
     const unsigned long long tag = omx_tag(ctx, F_MUON);
-    rc = s.bf16 ? run_muon<unsigned short>(ctx, t, n, rows, cols, s, static_cast<char*>(ws), L, tag)
-                : run_muon<float>(ctx, t, n, rows, cols, s, static_cast<char*>(ws), L, tag);
+    rc = s.bf16 ? run_muon<unsigned short>(ctx, t, n, rows, cols, s, static_cast<char*>(ws), L, list, tag)
+                : run_muon<float>(ctx, t, n, rows, cols, s, static_cast<char*>(ws), L, list, tag);
     if (rc != OMX_OK) return rc;
     first += n;
   }

@@ -202,6 +202,36 @@ def test_list_step_takes_the_scratch_there_is(be, rows, cols, count, room, bf16)
     small.close()
 
 
+@pytest.mark.parametrize("rows,cols,bf16", [(64, 48, 0), (130, 70, 1), (256, 256, 0), (256, 256, 1)])
+def test_list_step_refuses_each_matrix_by_itself(be, rows, cols, bf16):
+    """A gradient that is not finite, a momentum that is not, and a matrix whose norm overflows keep their own matrix as
+    it was; the others step as they do without them."""
+    from ojas_amd.backend import NON_FINITE, MuonNs5Config, OjasError
+
+    print(f"muon list refusals {rows}x{cols} bf16={bf16}", flush=True)
+    r = np.random.default_rng(rows)
+    ps, gs, ms = ([r.standard_normal((rows, cols)).astype(np.float32) * s for _ in range(6)] for s in (0.1, 0.05, 0.01))
+    bad_g, bad_m = [g.copy() for g in gs], [m.copy() for m in ms]
+    bad_g[0][3, 5] = np.nan
+    bad_m[2][-1, -1] = np.inf
+    bad_g[4][:] = 3e38
+    cfg = MuonNs5Config(0.02, 0.95, 0.1, 1, bf16)
+    out = []
+    for g, m in ((gs, ms), (bad_g, bad_m)):
+        dp, dg, dm = [be.upload(x) for x in ps], [be.upload(x) for x in g], [be.upload(x) for x in m]
+        be.muon_ns5_step_list(dp, dg, dm, cfg)
+        if g is bad_g:
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.code == NON_FINITE and "muon_ns5_step" in str(e.value)
+        out.append([(be.download(p), be.download(m)) for p, m in zip(dp, dm)])
+    for i in range(6):
+        if i in (0, 2, 4):
+            assert np.array_equal(out[1][i][0], ps[i]) and np.array_equal(out[1][i][1], bad_m[i]), i
+        else:
+            assert np.array_equal(out[1][i][0], out[0][i][0]) and np.array_equal(out[1][i][1], out[0][i][1]), i
+
+
 def test_a_model_of_many_matrices_steps_within_its_budget():
     """84 matrices of 512 x 512: 64 of them at once are 403 MB of scratch, one is 6.3."""
     from ojas_amd.backend import MiBackend
