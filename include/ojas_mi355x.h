@@ -282,7 +282,7 @@ int32_t omx_causal_attention_backward_saved(omx_ctx* ctx, const void* q, uint64_
                                             uint64_t window);
 
 /* causal_attention of the f32 tier, time-major as above: every tensor f32, head_dim 16 / 32 / 64 / 128 (other
- * shapes return Unsupported and the caller composes omx_permute_0213 with omx_causal_sdpa_*), pitches
+ * head dims return Unsupported and the caller composes omx_permute_0213 with omx_causal_sdpa_*), pitches
  * multiples of 4. lse is [batch, heads, time]. For a step driver that keeps q, k and v as column blocks of one
  * projection output. */
 int32_t omx_causal_attention_f32_forward(omx_ctx* ctx, const void* q, uint64_t q_pitch, const void* k,

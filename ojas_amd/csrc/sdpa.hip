@@ -41,6 +41,8 @@ constexpr int MAXD = 256;
 struct SdpaShape {
   int batch, heads, kv_heads, time, dim, window, rep;
   float scale;
+  // Element strides of a batch, a head and a row: q (and gq), k and v (and gk, gv), out (and gy). lse is [batch, heads, time].
+  long q_b, q_h, q_t, k_b, k_h, k_t, o_b, o_h, o_t;
 };
 
 __device__ __forceinline__ int first_key(const SdpaShape& s, int t) {
@@ -68,10 +70,10 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_fwd_rows_kernel(const TI* __r
   const int t = static_cast<int>(row % s.time);
   const long plane = row / s.time;
   const int h = static_cast<int>(plane % s.heads), b = static_cast<int>(plane / s.heads);
-  const long kv_plane = static_cast<long>(b) * s.kv_heads + h / s.rep;
-  const TI* qr = q + row * s.dim;
-  const TI* kh = k + kv_plane * s.time * s.dim;
-  const TI* vh = v + kv_plane * s.time * s.dim;
+  const long kv_plane = b * s.k_b + h / s.rep * s.k_h;
+  const TI* qr = q + b * s.q_b + h * s.q_h + t * s.q_t;
+  const TI* kh = k + kv_plane;
+  const TI* vh = v + kv_plane;
   const int D = s.dim;
   for (int d = lane; d < D; d += 64) q_lds[wave][d] = dev_load<TI>(qr, d);
   constexpr int ND = MAXD / 64;
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_fwd_rows_kernel(const TI* __r
     const int j = j0 + lane;
     float sc = -INFINITY;
     if (j < j_end) {
-      const TI* kr = kh + static_cast<long>(j) * D;
+      const TI* kr = kh + j * s.k_t;
       float dot = 0.0f;
       for (int d = 0; d < D; ++d) dot += q_lds[wave][d] * dev_load<TI>(kr, d);
       sc = dot * s.scale;
@@ -108,7 +110,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_fwd_rows_kernel(const TI* __r
       const int d = i * 64 + lane;
       if (d < D) {
         float a = acc[i] * rescale;
-        for (int jj = 0; jj < nk; ++jj) a += p_lds[wave][jj] * dev_load<TI>(vh, static_cast<long>(j0 + jj) * D + d);
+        for (int jj = 0; jj < nk; ++jj) a += p_lds[wave][jj] * dev_load<TI>(vh, (j0 + jj) * s.k_t + d);
         acc[i] = a;
       }
     }
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_fwd_rows_kernel(const TI* __r
   }
   bad |= !(dev_finite(run_sum) && run_sum > 0.0f);
   const float inv = 1.0f / run_sum;
-  TO* orow = out + row * D;
+  TO* orow = out + b * s.o_b + h * s.o_h + t * s.o_t;
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
     const int d = i * 64 + lane;
@@ -134,12 +136,14 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_fwd_rows_kernel(const TI* __r
 template <typename TOUT, typename TGY>
 __global__ __launch_bounds__(SD_THREADS) void sdpa_delta_kernel(const TOUT* __restrict__ out,
                                                                 const TGY* __restrict__ gy,
-                                                                float* __restrict__ delta, long rows, int D) {
+                                                                float* __restrict__ delta, SdpaShape s) {
   const int lane = threadIdx.x & 63;
   const long row = static_cast<long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  if (row >= static_cast<long>(s.batch) * s.heads * s.time) return;
+  const long plane = row / s.time;
+  const long at = plane / s.heads * s.o_b + plane % s.heads * s.o_h + row % s.time * s.o_t;
   float acc = 0.0f;
-  for (int d = lane; d < D; d += 64) acc += dev_load<TGY>(gy, row * D + d) * dev_load<TOUT>(out, row * D + d);
+  for (int d = lane; d < s.dim; d += 64) acc += dev_load<TGY>(gy, at + d) * dev_load<TOUT>(out, at + d);
   acc = wave_sum(acc);
   if (lane == 0) delta[row] = acc;
 }
@@ -173,13 +177,14 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dq_rows_kernel(
   const int t = static_cast<int>(row % s.time);
   const long plane = row / s.time;
   const int h = static_cast<int>(plane % s.heads), b = static_cast<int>(plane / s.heads);
-  const long kv_plane = static_cast<long>(b) * s.kv_heads + h / s.rep;
-  const TI* kh = k + kv_plane * s.time * s.dim;
-  const TI* vh = v + kv_plane * s.time * s.dim;
+  const long kv_plane = b * s.k_b + h / s.rep * s.k_h, q_row = b * s.q_b + h * s.q_h + t * s.q_t;
+  const long o_row = b * s.o_b + h * s.o_h + t * s.o_t;
+  const TI* kh = k + kv_plane;
+  const TI* vh = v + kv_plane;
   const int D = s.dim;
   for (int d = lane; d < D; d += 64) {
-    q_lds[wave][d] = dev_load<TI>(q, row * D + d);
-    g_lds[wave][d] = dev_load<TI>(gy, row * D + d);
+    q_lds[wave][d] = dev_load<TI>(q, q_row + d);
+    g_lds[wave][d] = dev_load<TI>(gy, o_row + d);
   }
   const float row_lse = lse[row], dr = delta[row];
   bool bad = !(dev_finite(row_lse) && dev_finite(dr));
@@ -192,8 +197,8 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dq_rows_kernel(
     const int j = j0 + lane;
     float coef = 0.0f;
     if (j < j_end) {
-      const TI* kr = kh + static_cast<long>(j) * D;
-      const TI* vr = vh + static_cast<long>(j) * D;
+      const TI* kr = kh + j * s.k_t;
+      const TI* vr = vh + j * s.k_t;
       float dot = 0.0f, dp = 0.0f;
       for (int d = 0; d < D; ++d) {
         dot += q_lds[wave][d] * dev_load<TI>(kr, d);
@@ -213,7 +218,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dq_rows_kernel(
       const int d = i * 64 + lane;
       if (d < D) {
         float a = acc[i];
-        for (int jj = 0; jj < nk; ++jj) a += c_lds[wave][jj] * dev_load<TI>(kh, static_cast<long>(j0 + jj) * D + d);
+        for (int jj = 0; jj < nk; ++jj) a += c_lds[wave][jj] * dev_load<TI>(kh, (j0 + jj) * s.k_t + d);
         acc[i] = a;
       }
     }
@@ -224,7 +229,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dq_rows_kernel(
     const int d = i * 64 + lane;
     if (d < D) {
       bad |= !dev_finite(acc[i]);
-      dev_store<TO>(gq, row * D + d, acc[i]);
+      dev_store<TO>(gq, q_row + d, acc[i]);
     }
   }
   if (bad) dev_raise_fault(fault, tag);
@@ -249,9 +254,10 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dkv_rows_kernel(
   const long kv_plane = row / s.time;
   const int g = static_cast<int>(kv_plane % s.kv_heads), b = static_cast<int>(kv_plane / s.kv_heads);
   const int D = s.dim;
+  const long k_row = b * s.k_b + g * s.k_h + j * s.k_t;
   for (int d = lane; d < D; d += 64) {
-    k_lds[wave][d] = dev_load<TI>(k, row * D + d);
-    v_lds[wave][d] = dev_load<TI>(v, row * D + d);
+    k_lds[wave][d] = dev_load<TI>(k, k_row + d);
+    v_lds[wave][d] = dev_load<TI>(v, k_row + d);
   }
   constexpr int ND = MAXD / 64;
   float acck[ND], accv[ND];
@@ -260,17 +266,17 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dkv_rows_kernel(
   bool bad = false;
   const int t_end = last_query(s, j) + 1;
   for (int r = 0; r < s.rep; ++r) {
-    const long q_plane = static_cast<long>(b) * s.heads + static_cast<long>(g) * s.rep + r;
-    const TI* qh = q + q_plane * s.time * D;
-    const TI* gh = gy + q_plane * s.time * D;
+    const long head = static_cast<long>(g) * s.rep + r, q_plane = static_cast<long>(b) * s.heads + head;
+    const TI* qh = q + b * s.q_b + head * s.q_h;
+    const TI* gh = gy + b * s.o_b + head * s.o_h;
     const float* lse_h = lse + q_plane * s.time;
     const float* del_h = delta + q_plane * s.time;
     for (int t0 = j; t0 < t_end; t0 += 64) {
       const int t = t0 + lane;
       float coef = 0.0f, p = 0.0f;
       if (t < t_end) {
-        const TI* qr = qh + static_cast<long>(t) * D;
-        const TI* gr = gh + static_cast<long>(t) * D;
+        const TI* qr = qh + t * s.q_t;
+        const TI* gr = gh + t * s.o_t;
         float dot = 0.0f, dp = 0.0f;
         for (int d = 0; d < D; ++d) {
           dot += dev_load<TI>(qr, d) * k_lds[wave][d];
@@ -292,8 +298,8 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dkv_rows_kernel(
         if (d < D) {
           float ak = acck[i], av = accv[i];
           for (int tt = 0; tt < nq; ++tt) {
-            ak += c_lds[wave][tt] * dev_load<TI>(qh, static_cast<long>(t0 + tt) * D + d);
-            av += p_lds[wave][tt] * dev_load<TI>(gh, static_cast<long>(t0 + tt) * D + d);
+            ak += c_lds[wave][tt] * dev_load<TI>(qh, (t0 + tt) * s.q_t + d);
+            av += p_lds[wave][tt] * dev_load<TI>(gh, (t0 + tt) * s.o_t + d);
           }
           acck[i] = ak;
           accv[i] = av;
@@ -307,8 +313,8 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dkv_rows_kernel(
     const int d = i * 64 + lane;
     if (d < D) {
       bad |= !(dev_finite(acck[i]) && dev_finite(accv[i]));
-      dev_store<TO>(gk, row * D + d, acck[i]);
-      dev_store<TO>(gv, row * D + d, accv[i]);
+      dev_store<TO>(gk, k_row + d, acck[i]);
+      dev_store<TO>(gv, k_row + d, accv[i]);
     }
   }
   if (bad) dev_raise_fault(fault, tag);
@@ -333,20 +339,23 @@ int32_t check_shape(omx_ctx* ctx, const char* op, uint64_t batch, uint64_t heads
   s->window = (window == 0 || window >= time) ? 0 : static_cast<int>(window);
   s->rep = static_cast<int>(heads / kv_heads);
   s->scale = 1.0f / sqrtf(static_cast<float>(static_cast<uint32_t>(dim)));
+  const long plane = static_cast<long>(time) * s->dim;  // contiguous [B, H, T, D]
+  s->q_t = s->k_t = s->o_t = s->dim;
+  s->q_h = s->k_h = s->o_h = plane;
+  s->q_b = s->o_b = plane * s->heads;
+  s->k_b = plane * s->kv_heads;
   return OMX_OK;
 }
 
-// Contiguous [B, H, T, D] tensors for the f32 matrix kernels.
+// The f32 matrix kernels' arguments.
 Sdpa32Args sdpa32_args(omx_ctx* ctx, const void* q, const void* k, const void* v, const SdpaShape& s, unsigned long long tag) {
   Sdpa32Args a{};
   a.q = static_cast<const float*>(q);
   a.k = k;
   a.v = v;
-  const long plane = static_cast<long>(s.time) * s.dim;
-  a.q_t = a.k_t = a.o_t = s.dim;
-  a.q_h = a.k_h = a.o_h = plane;
-  a.q_b = a.o_b = plane * s.heads;
-  a.k_b = plane * s.kv_heads;
+  a.q_b = s.q_b; a.q_h = s.q_h; a.q_t = s.q_t;
+  a.k_b = s.k_b; a.k_h = s.k_h; a.k_t = s.k_t;
+  a.o_b = s.o_b; a.o_h = s.o_h; a.o_t = s.o_t;
   a.kv_heads = s.kv_heads;
   a.rep = s.rep;
   a.tq = a.tk = a.capacity = s.time;
@@ -355,6 +364,39 @@ Sdpa32Args sdpa32_args(omx_ctx* ctx, const void* q, const void* k, const void* v
   a.fault = ctx->fault;
   a.tag = tag;
   return a;
+}
+
+// A wave per row: any head dim up to 256 and any number of planes.
+template <typename TI, typename TO>
+int32_t rows_forward(omx_ctx* ctx, const void* q, const void* k, const void* v, void* out, void* lse, const SdpaShape& s,
+                     unsigned long long tag) {
+  const long rows = static_cast<long>(s.batch) * s.heads * s.time;
+  omx_launch(ctx, (sdpa_fwd_rows_kernel<TI, TO>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(SD_THREADS), 0,
+             static_cast<const TI*>(q), static_cast<const TI*>(k), static_cast<const TI*>(v), static_cast<TO*>(out),
+             static_cast<float*>(lse), s, ctx->fault, tag);
+  OMX_LAUNCH_CHECK(ctx, "sdpa_fwd_rows_kernel");
+  return OMX_OK;
+}
+template <typename TOUT, typename TGY>
+int32_t rows_delta(omx_ctx* ctx, const void* out, const void* gy, float* delta, const SdpaShape& s) {
+  const long rows = static_cast<long>(s.batch) * s.heads * s.time;
+  omx_launch(ctx, (sdpa_delta_kernel<TOUT, TGY>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(SD_THREADS), 0,
+             static_cast<const TOUT*>(out), static_cast<const TGY*>(gy), delta, s);
+  OMX_LAUNCH_CHECK(ctx, "sdpa_delta_kernel");
+  return OMX_OK;
+}
+template <typename TI, typename TO>
+int32_t rows_backward(omx_ctx* ctx, const void* q, const void* k, const void* v, const float* lse, const float* delta, const void* gy,
+                      void* gq, void* gk, void* gv, const SdpaShape& s, unsigned long long tag) {
+  const long rows = static_cast<long>(s.batch) * s.heads * s.time, kv_rows = static_cast<long>(s.batch) * s.kv_heads * s.time;
+  const TI *tq = static_cast<const TI*>(q), *tk = static_cast<const TI*>(k), *tv = static_cast<const TI*>(v);
+  const TI* tg = static_cast<const TI*>(gy);
+  omx_launch(ctx, (sdpa_bwd_dq_rows_kernel<TI, TO>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(SD_THREADS), 0, tq, tk, tv, lse,
+             delta, tg, static_cast<TO*>(gq), s, ctx->fault, tag);
+  omx_launch(ctx, (sdpa_bwd_dkv_rows_kernel<TI, TO>), dim3(static_cast<unsigned>((kv_rows + 3) / 4)), dim3(SD_THREADS), 0, tq, tk, tv,
+             lse, delta, tg, static_cast<TO*>(gk), static_cast<TO*>(gv), s, ctx->fault, tag);
+  OMX_LAUNCH_CHECK(ctx, "sdpa backward row kernels");
+  return OMX_OK;
 }
 
 }  // namespace
@@ -383,19 +425,10 @@ int32_t omx_causal_sdpa_forward(omx_ctx* ctx, const void* q, const void* k, cons
     a.lse = static_cast<float*>(lse);
     return omx_sdpa32_forward(ctx, a, s.batch, s.dim, false);
   }
-  const long rows = static_cast<long>(batch) * heads * time;
-  dim3 grid(static_cast<unsigned>((rows + 3) / 4)), block(SD_THREADS);
-#define SDPA_FWD(TI, TO)                                                                                          \
-  omx_launch(ctx, (sdpa_fwd_rows_kernel<TI, TO>), grid, block, 0, static_cast<const TI*>(q),      \
-                     static_cast<const TI*>(k), static_cast<const TI*>(v), static_cast<TO*>(out),                 \
-                     static_cast<float*>(lse), s, ctx->fault, tag)
-  if (operand_dtype == OMX_F32 && out_dtype == OMX_F32) SDPA_FWD(float, float);
-  else if (operand_dtype == OMX_F32) SDPA_FWD(float, unsigned short);
-  else if (out_dtype == OMX_F32) SDPA_FWD(unsigned short, float);
-  else SDPA_FWD(unsigned short, unsigned short);
-#undef SDPA_FWD
-  OMX_LAUNCH_CHECK(ctx, "sdpa_fwd_rows_kernel");
-  return OMX_OK;
+  const auto rows = operand_dtype == OMX_F32 ? (out_dtype == OMX_F32 ? &rows_forward<float, float> : &rows_forward<float, unsigned short>)
+                    : out_dtype == OMX_F32   ? &rows_forward<unsigned short, float>
+                                             : &rows_forward<unsigned short, unsigned short>;
+  return rows(ctx, q, k, v, out, lse, s, tag);
 }
 
 int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, const void* v, const void* out,
@@ -444,12 +477,10 @@ int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, con
     return omx_flash_sdpa_backward(ctx, q, k, v, out16, residual, static_cast<const float*>(lse), gy16, gq, gk, gv,
                                    grad_dtype, batch, heads, kv_heads, time, head_dim, s.window, s.scale, tag, nullptr);
   }
-  const long kv_rows = static_cast<long>(batch) * kv_heads * time;
   void* ws = nullptr;
   rc = omx_workspace(ctx, rows * sizeof(float), &ws);
   if (rc != OMX_OK) return rc;
   float* delta = static_cast<float*>(ws);
-  dim3 grid(static_cast<unsigned>((rows + 3) / 4)), kv_grid(static_cast<unsigned>((kv_rows + 3) / 4)), block(SD_THREADS);
   const float* lsef = static_cast<const float*>(lse);
   const bool matrix = ctx->sdpa_tiled && operand_dtype == OMX_F32 && grad_dtype == OMX_F32 && gy_dtype == OMX_F32 &&
                       out_dtype == OMX_F32 && omx_sdpa32_supports(head_dim, batch * kv_heads, {q, k, v, out, gy, gq, gk, gv}, {});
@@ -466,15 +497,11 @@ int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, con
   }
   // The row term reads out and grad_output as they are stored; the two passes read grad_output in
   // the operands' storage type.
-#define SDPA_DELTA(TOUT, TGY)                                                                                 \
-  omx_launch(ctx, (sdpa_delta_kernel<TOUT, TGY>), grid, block, 0, static_cast<const TOUT*>(out), \
-                     static_cast<const TGY*>(gy), delta, rows, s.dim)
-  if (out_dtype == OMX_F32 && gy_dtype == OMX_F32) SDPA_DELTA(float, float);
-  else if (out_dtype == OMX_F32) SDPA_DELTA(float, unsigned short);
-  else if (gy_dtype == OMX_F32) SDPA_DELTA(unsigned short, float);
-  else SDPA_DELTA(unsigned short, unsigned short);
-#undef SDPA_DELTA
-  OMX_LAUNCH_CHECK(ctx, "sdpa_delta_kernel");
+  const auto row_term = out_dtype == OMX_F32 ? (gy_dtype == OMX_F32 ? &rows_delta<float, float> : &rows_delta<float, unsigned short>)
+                        : gy_dtype == OMX_F32 ? &rows_delta<unsigned short, float>
+                                              : &rows_delta<unsigned short, unsigned short>;
+  rc = row_term(ctx, out, gy, delta, s);
+  if (rc != OMX_OK) return rc;
   if (gy_dtype != operand_dtype) {
     void* conv = nullptr;
     rc = omx_workspace(ctx, n * omx_dtype_size(operand_dtype), &conv, 1);
@@ -483,22 +510,10 @@ int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, con
     if (rc != OMX_OK) return rc;
     gy = conv;
   }
-#define SDPA_BWD(TI, TO)                                                                                              \
-  do {                                                                                                                \
-    omx_launch(ctx, (sdpa_bwd_dq_rows_kernel<TI, TO>), grid, block, 0, static_cast<const TI*>(q),     \
-                       static_cast<const TI*>(k), static_cast<const TI*>(v), lsef, delta, static_cast<const TI*>(gy), \
-                       static_cast<TO*>(gq), s, ctx->fault, tag);                                                     \
-    omx_launch(ctx, (sdpa_bwd_dkv_rows_kernel<TI, TO>), kv_grid, block, 0,                            \
-                       static_cast<const TI*>(q), static_cast<const TI*>(k), static_cast<const TI*>(v), lsef, delta,  \
-                       static_cast<const TI*>(gy), static_cast<TO*>(gk), static_cast<TO*>(gv), s, ctx->fault, tag);   \
-  } while (0)
-  if (operand_dtype == OMX_F32 && grad_dtype == OMX_F32) SDPA_BWD(float, float);
-  else if (operand_dtype == OMX_F32) SDPA_BWD(float, unsigned short);
-  else if (grad_dtype == OMX_F32) SDPA_BWD(unsigned short, float);
-  else SDPA_BWD(unsigned short, unsigned short);
-#undef SDPA_BWD
-  OMX_LAUNCH_CHECK(ctx, "sdpa backward row kernels");
-  return OMX_OK;
+  const auto passes = operand_dtype == OMX_F32 ? (grad_dtype == OMX_F32 ? &rows_backward<float, float> : &rows_backward<float, unsigned short>)
+                      : grad_dtype == OMX_F32  ? &rows_backward<unsigned short, float>
+                                               : &rows_backward<unsigned short, unsigned short>;
+  return passes(ctx, q, k, v, lsef, delta, gy, gq, gk, gv, s, tag);
 }
 
 int32_t omx_causal_sdpa_backward_recompute(omx_ctx* ctx, const void* q, const void* k, const void* v, const void* gy,
@@ -633,28 +648,29 @@ int32_t omx_causal_attention_backward_saved(omx_ctx* ctx, const void* q, uint64_
                             gq, gk, gv, grad_dtype, batch, time, heads, kv_heads, head_dim, window);
 }
 
-static int32_t attention_f32(omx_ctx* ctx, const char* op, uint32_t fault, const void* q, uint64_t q_pitch, const void* k,
-                             const void* v, uint64_t kv_pitch, uint64_t out_pitch, uint64_t batch, uint64_t time, uint64_t heads,
-                             uint64_t kv_heads, uint64_t head_dim, uint64_t window, std::initializer_list<const void*> ptrs, Sdpa32Args* a) {
+// The shape with the time-major tensors' strides, or why there is none. `rows`: on the kernels of a wave per row (the option
+// "sdpa_tiled" 0, or more planes than a grid of the matrix kernels has).
+static int32_t attention_f32(omx_ctx* ctx, const char* op, uint64_t q_pitch, uint64_t kv_pitch, uint64_t out_pitch, uint64_t batch,
+                             uint64_t time, uint64_t heads, uint64_t kv_heads, uint64_t head_dim, uint64_t window,
+                             std::initializer_list<const void*> ptrs, SdpaShape* s, bool* rows) {
   for (const void* p : ptrs)
     if (!p) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
-  SdpaShape s;
-  int32_t rc = check_shape(ctx, op, batch, heads, kv_heads, time, head_dim, window, &s);
+  int32_t rc = check_shape(ctx, op, batch, heads, kv_heads, time, head_dim, window, s);
   if (rc != OMX_OK) return rc;
   if (q_pitch < heads * head_dim || out_pitch < heads * head_dim || kv_pitch < kv_heads * head_dim)
     return omx_fail(ctx, OMX_SHAPE, "%s: row pitch below heads * head_dim", op);
   const long qp = static_cast<long>(q_pitch), kp = static_cast<long>(kv_pitch), op_ = static_cast<long>(out_pitch);
-  if (!omx_sdpa32_supports(head_dim, batch * kv_heads, ptrs, {qp, kp, op_}))
+  if (!omx_sdpa32_supports(head_dim, 1, ptrs, {qp, kp, op_}))
     return omx_fail(ctx, OMX_UNSUPPORTED, "%s: head_dim %llu (16, 32, 64 or 128), 16-byte aligned tensors and pitches", op,
                     (unsigned long long)head_dim);
-  *a = sdpa32_args(ctx, q, k, v, s, omx_tag(ctx, fault));
-  a->q_h = a->k_h = a->o_h = s.dim;
-  a->q_t = qp;
-  a->k_t = kp;
-  a->o_t = op_;
-  a->q_b = qp * s.time;
-  a->k_b = kp * s.time;
-  a->o_b = op_ * s.time;
+  *rows = !ctx->sdpa_tiled || !omx_sdpa32_supports(head_dim, batch * kv_heads, ptrs, {qp, kp, op_});
+  s->q_h = s->k_h = s->o_h = s->dim;
+  s->q_t = qp;
+  s->k_t = kp;
+  s->o_t = op_;
+  s->q_b = qp * s->time;
+  s->k_b = kp * s->time;
+  s->o_b = op_ * s->time;
   return OMX_OK;
 }
 
@@ -662,10 +678,14 @@ int32_t omx_causal_attention_f32_forward(omx_ctx* ctx, const void* q, uint64_t q
                                          void* out, uint64_t out_pitch, void* lse, uint64_t batch, uint64_t time, uint64_t heads,
                                          uint64_t kv_heads, uint64_t head_dim, uint64_t window) {
   OMX_REQUIRE_CTX(ctx);
-  Sdpa32Args a;
-  int32_t rc = attention_f32(ctx, "causal_attention_f32_forward", F_SDPA_FORWARD, q, q_pitch, k, v, kv_pitch, out_pitch, batch, time, heads,
-                             kv_heads, head_dim, window, {q, k, v, out, lse}, &a);
+  SdpaShape s;
+  bool rows;
+  int32_t rc = attention_f32(ctx, "causal_attention_f32_forward", q_pitch, kv_pitch, out_pitch, batch, time, heads, kv_heads, head_dim,
+                             window, {q, k, v, out, lse}, &s, &rows);
   if (rc != OMX_OK) return rc;
+  const unsigned long long tag = omx_tag(ctx, F_SDPA_FORWARD);
+  if (rows) return rows_forward<float, float>(ctx, q, k, v, out, lse, s, tag);
+  Sdpa32Args a = sdpa32_args(ctx, q, k, v, s, tag);
   a.out = static_cast<float*>(out);
   a.lse = static_cast<float*>(lse);
   return omx_sdpa32_forward(ctx, a, static_cast<int>(batch), static_cast<int>(head_dim), false);
@@ -676,13 +696,21 @@ int32_t omx_causal_attention_f32_backward(omx_ctx* ctx, const void* q, uint64_t 
                                           uint64_t batch, uint64_t time, uint64_t heads, uint64_t kv_heads, uint64_t head_dim,
                                           uint64_t window) {
   OMX_REQUIRE_CTX(ctx);
-  Sdpa32Args a;
-  int32_t rc = attention_f32(ctx, "causal_attention_f32_backward", F_SDPA_BACKWARD, q, q_pitch, k, v, kv_pitch, out_pitch, batch, time,
-                             heads, kv_heads, head_dim, window, {q, k, v, out, gy, lse, gq, gk, gv}, &a);
+  SdpaShape s;
+  bool rows;
+  int32_t rc = attention_f32(ctx, "causal_attention_f32_backward", q_pitch, kv_pitch, out_pitch, batch, time, heads, kv_heads, head_dim,
+                             window, {q, k, v, out, gy, lse, gq, gk, gv}, &s, &rows);
   if (rc != OMX_OK) return rc;
   void* ws = nullptr;
   rc = omx_workspace(ctx, batch * heads * time * sizeof(float), &ws);
   if (rc != OMX_OK) return rc;
+  const unsigned long long tag = omx_tag(ctx, F_SDPA_BACKWARD);
+  if (rows) {
+    rc = rows_delta<float, float>(ctx, out, gy, static_cast<float*>(ws), s);
+    if (rc != OMX_OK) return rc;
+    return rows_backward<float, float>(ctx, q, k, v, static_cast<const float*>(lse), static_cast<const float*>(ws), gy, gq, gk, gv, s, tag);
+  }
+  Sdpa32Args a = sdpa32_args(ctx, q, k, v, s, tag);
   a.out = const_cast<float*>(static_cast<const float*>(out));  // read only
   a.lse = const_cast<float*>(static_cast<const float*>(lse));
   a.gy = static_cast<const float*>(gy);

@@ -243,3 +243,13 @@ def test_hybrid_step_muon_on_matrices_adamw_on_tables_and_norms(be, bf16):
     losses = [tr.step_hybrid(muon, adamw, 1.0)[0] for _ in range(8)]
     assert losses[-1] < step_loss and tr.steps() == 9
     tr.close()
+
+
+def test_f32_step_of_more_sequences_and_heads_than_a_grid_axis_holds(be):
+    """65600 (sequence, head) planes of two tokens each: attention leaves the matrix kernels, the step runs."""
+    print("gpt f32 step, 65600 attention planes", flush=True)
+    tr, _, (loss, grads), (oloss, ograds) = run_case(be, (1, 64, 4, 16, 128, 2, 50, 16400, 0, 0), 5, 0.1)
+    assert abs(loss - oloss) <= 1e-5 * abs(oloss), (loss, oloss)
+    for i, (g, og) in enumerate(zip(grads, ograds)):
+        assert float(np.max(np.abs(g - og))) <= 1e-4 * float(np.max(np.abs(og))), i
+    tr.close()

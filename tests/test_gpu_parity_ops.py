@@ -496,6 +496,46 @@ def test_causal_sdpa_f32_tiled_kernels_agree_with_the_row_kernels(be, shape, hkv
             close(a, c, F32_TOL, "tiled against the oracle: " + name)
 
 
+@pytest.mark.parametrize("b,h,hkv,t,d,window,tiled", [(2, 4, 2, 70, 64, 0, 0), (1, 3, 3, 130, 16, 40, 0), (2, 2, 1, 65, 128, 0, 0),
+                                                    (16500, 4, 4, 3, 16, 0, 1), (8200, 8, 8, 2, 32, 1, 1)])
+def test_time_major_f32_attention_takes_the_row_kernels_where_it_must(be, b, h, hkv, t, d, window, tiled):
+    """`omx_causal_attention_f32_*` with "sdpa_tiled" 0, and over more (batch, KV head) planes than a grid axis of the matrix
+    kernels holds: the bits of the row kernels on permuted tensors, whatever lies between a row's end and its pitch."""
+    import ctypes as C
+
+    from ojas_amd.backend import F32
+
+    print(f"time-major f32 attention on rows {b} {h}/{hkv} {t} {d} window {window} tiled {tiled}", flush=True)
+    r = np.random.default_rng(b + t)
+    pitch, op = (h + 2 * hkv) * d + 4, h * d + 8
+    qkv = r.standard_normal((b, t, pitch)).astype(np.float32)
+    gy = r.standard_normal((b, t, op)).astype(np.float32)
+    cut = lambda x, at, n: np.ascontiguousarray(x[:, :, at:at + n * d].reshape(b, t, n, d).transpose(0, 2, 1, 3))
+    q, k, v, g = cut(qkv, 0, h), cut(qkv, h * d, hkv), cut(qkv, (h + hkv) * d, hkv), cut(gy, 0, h)
+    dqkv, dgy = be.upload(qkv), be.upload(gy)
+    out, grad, lse = be.zeros((b, t, op)), be.zeros((b, t, pitch)), be.empty((b, h, t))
+    at = lambda x, n: C.c_void_p(x.ptr + 4 * n)
+    u = C.c_uint64
+    dims = [u(x) for x in (b, t, h, hkv, d, window)]
+    ins = [at(dqkv, 0), u(pitch), at(dqkv, h * d), at(dqkv, (h + hkv) * d), u(pitch)]
+    try:
+        be.set_option("sdpa_tiled", tiled)
+        be._check(be._lib.omx_causal_attention_f32_forward(be._ctx, *ins, at(out, 0), u(op), at(lse, 0), *dims))
+        be._check(be._lib.omx_causal_attention_f32_backward(be._ctx, *ins, at(out, 0), at(dgy, 0), u(op), at(lse, 0), at(grad, 0),
+                                                            at(grad, h * d), at(grad, (h + hkv) * d), *dims))
+        be.set_option("sdpa_tiled", 0)
+        up = [be.upload(x) for x in (q, k, v, g)]
+        y, l = be.causal_sdpa_forward(*up[:3], window or None, F32)
+        grads = be.causal_sdpa_backward(*up[:3], y, l, up[3], window or None, F32)
+    finally:
+        be.set_option("sdpa_tiled", 1)
+    got, ggot = be.download(out), be.download(grad)
+    assert np.array_equal(cut(got, 0, h), be.download(y)) and np.array_equal(be.download(lse), be.download(l))
+    assert not got[:, :, h * d:].any() and not ggot[:, :, pitch - 4:].any()
+    for x, start, n in zip(grads, (0, h * d, (h + hkv) * d), (h, hkv, hkv)):
+        assert np.array_equal(cut(ggot, start, n), be.download(x))
+
+
 def test_causal_sdpa_f32_with_more_planes_than_a_grid_axis_holds(be):
     """65536 (batch, head) planes of a short sequence: above the 65535 a grid's second axis takes,
     so the call goes to the row kernels (decided on the host) instead of failing at launch."""
