@@ -11,6 +11,7 @@
 // moments live in flat f32 arenas (one clip pass and one AdamW pass cover every
 // tensor), the bf16 tier keeps a bf16 mirror of the parameters that AdamW
 // refreshes, and saved activations have one slot per layer.
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -77,7 +78,8 @@ struct ogpt {
   // With the fused projection, the four weight gradients of every layer wait until the backward's
   // end: each layer's inputs (h1, ap, h2, g) and output gradients (below) sit at a fixed stride in
   // stacked buffers, the gradient arena holds the layers at a fixed stride too, and four strided-
-  // batch products over the layers replace 4 x layers split-K products.
+  // batch products over the layers replace 4 x layers split-K products. Where memory for all of them is refused, at
+  // creation or to an op of the step for its scratch, every layer forms its own again.
   bool deferred_dw = false;
   void *h1_all = nullptr, *ap_all = nullptr, *h2_all = nullptr, *g_all = nullptr;
   void *gu_all = nullptr, *gqkv_all = nullptr;  // [layers][N,mlp], [layers][N,3d] AD
@@ -118,6 +120,34 @@ int32_t alloc_t(ogpt* t, uint64_t count, T** out) {
   return OMX_OK;
 }
 int32_t alloc_act(ogpt* t, uint64_t count, void** out) { return alloc(t, count * t->asz, out); }
+void release(ogpt* t, void** p, uint64_t bytes) {
+  if (!*p) return;
+  (void)omx_free(t->ctx, *p);
+  t->owned.erase(std::find(t->owned.begin(), t->owned.end(), *p));
+  t->device_bytes -= bytes;
+  *p = nullptr;
+}
+
+// Gives up the buffers of the deferred weight gradients' output sides (9 N d elements for each layer at mlp = 4 d, which no
+// other path needs) for one layer's worth: every weight gradient is formed in its layer then.
+int32_t form_in_layer(ogpt* t) {
+  const uint64_t n = t->c.layers * t->N * t->asz, d = t->c.d_model, M = t->c.mlp;
+  release(t, &t->gu_all, n * M);
+  release(t, &t->gqkv_all, n * 3 * d);
+  release(t, &t->gyd_all, n * d);
+  release(t, &t->gyo_all, n * d);
+  t->deferred_dw = false;
+  TRY(alloc_act(t, t->N * M, &t->gu));
+  return alloc_act(t, t->N * 3 * d, &t->gqkv);
+}
+// `run`, which can start over; where it is refused for want of memory, once more without the deferred buffers.
+template <typename F>
+int32_t with_room(ogpt* t, F run) {
+  int32_t rc = run();
+  if (rc != OMX_CAPACITY_EXCEEDED || !t->deferred_dw) return rc;
+  TRY(form_in_layer(t));
+  return run();
+}
 
 // AD copy of an f32 tensor: the f32 tier aliases it, the bf16 tier rounds it.
 int32_t to_operand(ogpt* t, const float* src, void* scratch, uint64_t n, const void** out) {
@@ -295,14 +325,16 @@ int32_t backward(ogpt* t) {
   return OMX_OK;
 }
 
-}  // namespace
+// The loss and every gradient of the batch.
+int32_t gradients(ogpt* t) {
+  return with_room(t, [&] {
+    TRY(forward(t));
+    return backward(t);
+  });
+}
 
-extern "C" {
-
-int32_t ogpt_create(omx_ctx* ctx, const ogpt_config* config, ogpt** out) {
-  if (!ctx || !config || !out) return OMX_BACKEND;
-  *out = nullptr;
-  const ogpt_config& c = *config;
+// `defer`: with the weight gradients deferred where the model allows.
+int32_t create(omx_ctx* ctx, const ogpt_config& c, bool defer, ogpt** out) {
   if (c.d_model == 0 || c.heads == 0 || c.head_dim == 0 || c.mlp == 0 || c.ctx == 0 || c.vocab == 0 || c.batch == 0)
     return OMX_SHAPE;
   if (static_cast<uint64_t>(c.heads) * c.head_dim != c.d_model) return OMX_SHAPE;
@@ -381,7 +413,7 @@ int32_t ogpt_create(omx_ctx* ctx, const ogpt_config* config, ogpt** out) {
     CREATE_TRY(omx_upload(ctx, t->positions, 0, pos.data(), N * 4));
   }
   t->layers.resize(c.layers);
-  t->deferred_dw = t->fused_qkv && c.layers > 1;
+  t->deferred_dw = defer && t->fused_qkv && c.layers > 1;
   const uint64_t L = c.layers;
   if (t->deferred_dw) {
     CREATE_TRY(alloc_act(t, L * N * d, &t->h1_all));
@@ -450,6 +482,17 @@ int32_t ogpt_create(omx_ctx* ctx, const ogpt_config* config, ogpt** out) {
 #undef CREATE_TRY
   *out = t;
   return OMX_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int32_t ogpt_create(omx_ctx* ctx, const ogpt_config* config, ogpt** out) {
+  if (!ctx || !config || !out) return OMX_BACKEND;
+  *out = nullptr;
+  const int32_t rc = create(ctx, *config, true, out);
+  return rc == OMX_CAPACITY_EXCEEDED ? create(ctx, *config, false, out) : rc;
 }
 
 void ogpt_destroy(ogpt* t) {
@@ -527,8 +570,7 @@ int32_t ogpt_set_batch(ogpt* t, const uint32_t* ids, const uint32_t* targets) {
 
 int32_t ogpt_loss_and_grads(ogpt* t, float* loss) {
   if (!t) return OMX_BACKEND;
-  TRY(forward(t));
-  TRY(backward(t));
+  TRY(gradients(t));
   float l = 0.0f;
   TRY(omx_read_scalar_f32(t->ctx, t->loss, &l));
   if (loss) *loss = l;
@@ -558,8 +600,7 @@ static int32_t read_loss_and_flag(ogpt* t, float* loss) {
 
 int32_t ogpt_step(ogpt* t, const omx_adamw_config* adamw, float grad_clip, float* loss, float* grad_norm) {
   if (!t || !adamw) return OMX_BACKEND;
-  TRY(forward(t));
-  TRY(backward(t));
+  TRY(gradients(t));
   // Sync point 1: the global gradient norm is a host value (trainer.rs:821-824).
   void* grads[1] = {t->g32};
   uint64_t lens[1] = {t->P};
@@ -586,8 +627,7 @@ int32_t ogpt_step(ogpt* t, const omx_adamw_config* adamw, float grad_clip, float
 int32_t ogpt_step_hybrid(ogpt* t, const omx_muon_config* muon, const omx_adamw_config* adamw, float grad_clip,
                          float* loss, float* grad_norm) {
   if (!t || !muon || !adamw) return OMX_BACKEND;
-  TRY(forward(t));
-  TRY(backward(t));
+  TRY(gradients(t));
   void* grads[1] = {t->g32};
   uint64_t lens[1] = {t->P};
   float norm = 0.0f;
@@ -621,8 +661,10 @@ int32_t ogpt_step_hybrid(ogpt* t, const omx_muon_config* muon, const omx_adamw_c
     add(groups[2], t->li(l, 7));
   }
   for (Group& grp : groups)
-    TRY(omx_muon_ns5_step_batched(t->ctx, grp.p.data(), grp.g.data(), grp.m.data(), mirror ? grp.p16.data() : nullptr,
-                                  grp.p.size(), grp.rows, grp.cols, muon));
+    TRY(with_room(t, [&] {
+      return omx_muon_ns5_step_batched(t->ctx, grp.p.data(), grp.g.data(), grp.m.data(), mirror ? grp.p16.data() : nullptr,
+                                       grp.p.size(), grp.rows, grp.cols, muon);
+    }));
   float l = 0.0f;
   TRY(read_loss_and_flag(t, &l));
   t->tracked = ogpt::kHybrid;  // the matrices and their first-moment slots are Muon's from here on

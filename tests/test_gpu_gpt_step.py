@@ -253,3 +253,43 @@ def test_f32_step_of_more_sequences_and_heads_than_a_grid_axis_holds(be):
     for i, (g, og) in enumerate(zip(grads, ograds)):
         assert float(np.max(np.abs(g - og))) <= 1e-4 * float(np.max(np.abs(og))), i
     tr.close()
+
+
+@pytest.mark.parametrize("bf16,head_dim", [(0, 64), (1, 128)])
+@pytest.mark.parametrize("short", ["at creation", "in the step"])
+def test_weight_gradients_are_formed_layer_by_layer_where_memory_is_short(bf16, head_dim, short):
+    """A budget that lacks the room for every layer's output gradients (9 N d elements each), or has just that and none for
+    the scratch of the step's ops: the step runs, with the same loss and the same gradients up to the order of their sums
+    (f32: 1e-5 normwise; bf16 the same products in f32 accumulators, rounded nowhere else)."""
+    from ojas_amd.backend import AdamWConfig, MiBackend, MuonNs5Config
+    from ojas_amd.trainer import GptConfig, GptTrainer, synthetic_batch
+
+    layers, d, ctx, batch = 6, 256, 256, 12
+    print(f"gpt step, memory short {short}, bf16={bf16}", flush=True)
+    cfg = GptConfig(layers, d, d // head_dim, head_dim, 4 * d, ctx, 512, batch, 0, bf16)
+    ids, targets = synthetic_batch(cfg, 3)
+
+    def run(budget):
+        be = MiBackend(0, budget_bytes=budget)
+        tr = GptTrainer(be, cfg)
+        created = be.budget()["live"]
+        tr.set_params(make_params(tr.param_lens(), d, 3))
+        tr.set_batch(ids, targets)
+        loss, grads = tr.loss_and_grads(), tr.grads()
+        step = tr.step(AdamWConfig.nanolab(3e-4, 0.1), 1.0)
+        hybrid = tr.step_hybrid(MuonNs5Config(0.02, 0.95, 0.1, 1, bf16), AdamWConfig.nanolab(3e-4, 0.1), 1.0)
+        peak = be.budget()["peak"]
+        tr.close()
+        be.close()
+        return loss, grads, step + hybrid, created, peak
+
+    loss, grads, steps, created, peak = run(0)
+    size = 2 if bf16 else 4
+    kept = batch * ctx * size * (layers * 9 * d - 7 * d)  # the deferred buffers less one layer's
+    assert kept > peak - created + (16 << 20) > 17 << 20  # more than the scratch of the ops beside what is created
+    least = peak - kept + (8 << 20)
+    loss2, grads2, steps2, _, peak2 = run(min(least, created - 1) if short == "at creation" else max(least, created + (1 << 20)))
+    assert loss2 == loss and peak2 < peak
+    for i, (a, b) in enumerate(zip(grads2, grads)):
+        assert float(np.linalg.norm(a - b)) <= 1e-5 * float(np.linalg.norm(b)), i
+    assert np.allclose(steps2, steps, rtol=1e-4 if not bf16 else 1e-2)
