@@ -401,7 +401,8 @@ int32_t omx_adamw_step_bounded(omx_ctx* ctx, void* param_f32, const void* grad_f
                                const omx_adamw_config* config, void* param_bf16,
                                int32_t inputs_bounded, void* unbounded_flag);
 /* omx_adamw_step on `count` tensors in one set of launches (a small model's tens of vectors), bit for bit what
- * a call for each gives: each tensor is all-or-nothing by itself. The arrays hold device pointers. */
+ * a call for each gives, in the list's order where tensors overlap: each tensor is all-or-nothing by itself. The arrays
+ * hold device pointers. */
 int32_t omx_adamw_step_batched(omx_ctx* ctx, void* const* params_f32, const void* const* grads_f32,
                                void* const* moments1_f32, void* const* moments2_f32, const uint64_t* lens,
                                uint64_t count, uint64_t step, const omx_adamw_config* config);
@@ -426,7 +427,7 @@ int32_t omx_muon_ns5_step_batched(omx_ctx* ctx, void* const* params_f32, const v
                                   uint64_t rows, uint64_t cols, const omx_muon_config* config);
 /* omx_muon_ns5_step on each tensor of a list of one shape, in as few sets of launches as its scratch allows: 256 MiB at
  * most, as much of that as the budget has room for, and omx_muon_ns5_step's at least. Each tensor is all-or-nothing by
- * itself. */
+ * itself. The tensors of the list do not overlap. */
 int32_t omx_muon_ns5_step_list(omx_ctx* ctx, void* const* params_f32, const void* const* grads_f32,
                                void* const* momenta_f32, void* const* params_bf16, uint64_t count,
                                uint64_t rows, uint64_t cols, const omx_muon_config* config);
@@ -435,7 +436,7 @@ int32_t omx_muon_ns5_step_list(omx_ctx* ctx, void* const* params_f32, const void
 uint64_t omx_muon_scratch_bytes(uint64_t rows, uint64_t cols);
 /* BackendFloat::clip_grad_norm (backend.rs:1466-1471): global L2 norm with an
  * f64 sum of squares, returned on the host; scales in place when the clip
- * coefficient (clip_scale, backend.rs:277-303) is below 1. A sync point. */
+ * coefficient (clip_scale, backend.rs:277-303) is below 1 (a tensor that is listed twice, twice). A sync point. */
 int32_t omx_clip_grad_norm(omx_ctx* ctx, void* const* grads_f32, const uint64_t* lens,
                            uint64_t count, float max_norm, float* norm_out);
 
@@ -447,7 +448,8 @@ int32_t omx_residual_add(omx_ctx* ctx, const void* x, int32_t x_dtype, const voi
                          void* out, int32_t out_dtype, uint64_t n);
 /* BackendFloat::accumulate_grad / scale_grad (backend.rs:1473-1510). */
 int32_t omx_accumulate_grad(omx_ctx* ctx, void* acc_f32, const void* grad_f32, uint64_t n);
-/* omx_accumulate_grad on `count` pairs in one launch. */
+/* omx_accumulate_grad on `count` pairs, in one launch as far as no accumulator overlaps another pair's tensors (those
+ * follow in the list's order). */
 int32_t omx_accumulate_grads(omx_ctx* ctx, void* const* accs_f32, const void* const* grads_f32, const uint64_t* lens,
                              uint64_t count);
 int32_t omx_scale_grad(omx_ctx* ctx, void* grad_f32, float scale, uint64_t n);

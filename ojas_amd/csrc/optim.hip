@@ -10,6 +10,7 @@
 // Each element pass reads and writes every word once with 16-byte accesses.
 // An optimizer step is all-or-nothing: a check pass decides on the device,
 // and the apply pass writes nothing when any value of the call is non-finite.
+#include <algorithm>
 #include <cmath>
 
 #include "omx_common.h"
@@ -373,6 +374,30 @@ inline uint64_t fill_spans(TensorSpans& s, const uint64_t* lens, uint64_t count,
   return t;
 }
 
+// A list's tensors step side by side, so one that overlaps another's result has to wait for the next launch, as it would
+// for the next call. What the entries of a list read and write:
+struct Touched {
+  struct Span {
+    uintptr_t begin, end;
+    uint64_t entry;
+    bool write;
+  } spans[4 * LIST_MAX];
+  int count = 0;
+  void add(const void* p, uint64_t floats, uint64_t entry, bool write) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+    spans[count++] = Span{at, at + floats * sizeof(float), entry, write};
+  }
+  // How many of the first `took` entries can step side by side (one at least).
+  uint64_t apart(uint64_t took) {
+    std::sort(spans, spans + count, [](const Span& a, const Span& b) { return a.begin < b.begin; });
+    for (int i = 0; i < count; ++i)
+      for (int j = i + 1; j < count && spans[j].begin < spans[i].end; ++j)
+        if (spans[i].entry != spans[j].entry && (spans[i].write || spans[j].write))
+          took = std::min(took, std::max(spans[i].entry, spans[j].entry));
+    return took;
+  }
+};
+
 inline unsigned grid_for(uint64_t n, int cu_count) {
   uint64_t blocks = (n + OPT_THREADS * 4 - 1) / (OPT_THREADS * 4);
   uint64_t cap = static_cast<uint64_t>(cu_count > 0 ? cu_count : 256) * 16;
@@ -507,7 +532,13 @@ int32_t omx_adamw_step_batched(omx_ctx* ctx, void* const* params, const void* co
   if (rc != OMX_OK) return rc;
   for (uint64_t t = 0; t < count;) {
     AdamList list;
-    const uint64_t took = fill_spans(list.spans, lens + t, count - t, OPT_THREADS * 4);
+    uint64_t took = fill_spans(list.spans, lens + t, count - t, OPT_THREADS * 4);
+    Touched touched;
+    for (uint64_t i = 0; i < took; ++i) {
+      for (const void* p : {params[t + i], moments1[t + i], moments2[t + i]}) touched.add(p, lens[t + i], i, true);
+      touched.add(grads[t + i], lens[t + i], i, false);
+    }
+    list.spans.count = static_cast<int>(took = touched.apart(took));
     for (uint64_t i = 0; i < took; ++i) {
       list.p[i] = static_cast<float*>(params[t + i]);
       list.g[i] = static_cast<const float*>(grads[t + i]);
@@ -535,7 +566,13 @@ int32_t omx_accumulate_grads(omx_ctx* ctx, void* const* accs, const void* const*
   }
   for (uint64_t t = 0; t < count;) {
     AccumulateList list;
-    const uint64_t took = fill_spans(list.spans, lens + t, count - t, OPT_THREADS * 4);
+    uint64_t took = fill_spans(list.spans, lens + t, count - t, OPT_THREADS * 4);
+    Touched touched;
+    for (uint64_t i = 0; i < took; ++i) {
+      touched.add(accs[t + i], lens[t + i], i, true);
+      touched.add(grads[t + i], lens[t + i], i, false);
+    }
+    list.spans.count = static_cast<int>(took = touched.apart(took));
     for (uint64_t i = 0; i < took; ++i) {
       list.acc[i] = static_cast<float*>(accs[t + i]);
       list.grad[i] = static_cast<const float*>(grads[t + i]);
@@ -591,9 +628,12 @@ int32_t omx_clip_grad_norm(omx_ctx* ctx, void* const* grads, const uint64_t* len
   if (std::isnan(coef)) return omx_fail(ctx, OMX_NON_FINITE, "%s", op);
   if (coef > 1.0f) coef = 1.0f;
   if (coef < 1.0f) {
-    for (uint64_t t = 0; t < count;) {
+      for (uint64_t t = 0; t < count;) {
       ScaleList list;
-      const uint64_t took = fill_spans(list.spans, lens + t, count - t, OPT_THREADS * 4);
+      uint64_t took = fill_spans(list.spans, lens + t, count - t, OPT_THREADS * 4);
+      Touched touched;
+      for (uint64_t i = 0; i < took; ++i) touched.add(grads[t + i], lens[t + i], i, true);
+      list.spans.count = static_cast<int>(took = touched.apart(took));
       for (uint64_t i = 0; i < took; ++i) list.x[i] = static_cast<float*>(grads[t + i]);
       omx_launch(ctx, scale_list_kernel, dim3(list.spans.first[took]), dim3(OPT_THREADS), 0, list, coef);
       OMX_LAUNCH_CHECK(ctx, "scale_list_kernel");

@@ -656,6 +656,49 @@ def test_adamw_config_refusals(be):
     assert e.value.code == OUT_OF_RANGE
 
 
+@pytest.mark.parametrize("n", [5, 4096, 30000])
+def test_lists_that_name_a_tensor_twice_step_it_in_order(be, n):
+    """A tensor that a list writes twice, or writes and reads elsewhere (whole, or as a view of a part): what calls one
+    after the other give."""
+    from ojas_amd.backend import AdamWConfig, DeviceTensor
+
+    print(f"lists with repeated tensors {n}", flush=True)
+    r = np.random.default_rng(n)
+    x, y, z = (r.standard_normal(n).astype(np.float32) for _ in range(3))
+    view = lambda t, at, m: DeviceTensor(be, t.ptr + 4 * at, (m,), t.dtype, owns=False)
+    half = (n // 2 + 3) // 4 * 4 if n > 8 else 2
+    # clip_grad_norm: counted and scaled as often as it is listed
+    dx, dy = be.upload(x), be.upload(y)
+    norm = be.clip_grad_norm([dx, dy, dx, view(dx, half, n - half)], 0.5)
+    want = np.sqrt(sum(float((v.astype(np.float64) ** 2).sum()) for v in (x, y, x, x[half:])))
+    assert abs(norm - want) <= 1e-6 * want
+    coef = np.float32(np.float32(0.5) / (np.float32(norm) + np.float32(1e-6)))
+    twice = (x * coef) * coef
+    twice[half:] *= coef
+    assert np.array_equal(be.download(dx), twice) and np.array_equal(be.download(dy), y * coef)
+    # accumulate_grads: a repeated accumulator, an accumulator that is the next one's gradient, a view of one
+    dx, dy, dz = be.upload(x), be.upload(y), be.upload(z)
+    be.accumulate_grads([dx, dx, dy, view(dx, 0, half)], [dz, dy, dx, view(dz, 0, half)])
+    wx = (x + z) + y
+    wy = y + wx
+    wx[:half] += z[:half]
+    assert np.array_equal(be.download(dx), wx) and np.array_equal(be.download(dy), wy)
+    # adamw_step_batched: one parameter and its moments twice, a parameter that is another's gradient
+    cfg = AdamWConfig(1e-2, 0.9, 0.95, 1e-8, 0.1)
+
+    def tensors():
+        return [be.upload(t) for t in (x, y, z, np.abs(x), np.abs(y), np.abs(z))]
+
+    p, g, q, m, v, w = tensors()
+    be.adamw_step_batched([p, p, q], [g, g, p], [m, m, g], [v, v, w], 3, cfg)
+    got = [be.download(t) for t in (p, m, v, q, g, w)]
+    p, g, q, m, v, w = tensors()
+    for args in ((p, g, m, v), (p, g, m, v), (q, p, g, w)):
+        be.adamw_step(*args, 3, cfg)
+    for a, b in zip(got, (p, m, v, q, g, w)):
+        assert np.array_equal(a, be.download(b))
+
+
 def test_clip_grad_norm(be):
     r = orc.SplitMix64(11)
     grads = [r.vec(n, 1.0) for n in (1, 1000, 70_001, 300_000)]
