@@ -558,13 +558,32 @@ class MiBackend(_native.Methods):
     def adamw_step_batched(self, params, grads, moments1, moments2, step: int, config: AdamWConfig):
         """`adamw_step` on several tensors in one set of launches (in place, each all-or-nothing by itself)."""
         lists = (params, grads, moments1, moments2)
-        for p, g, m1, m2 in zip(*lists):
-            shapes.adamw_step_dims(p, g, m1, m2)
-        if len({len(ts) for ts in lists}) != 1:
-            raise OjasError(SHAPE, "adamw_step_batched: one gradient and two moments for each parameter")
+        self._check_lists("adamw_step", shapes.adamw_step_dims, lists)
         tables = [self._pointers(ts) for ts in lists]
         _native.omx_adamw_step_batched(self._context, *[C.addressof(t) for t in tables],
                                        C.addressof(lens := self._lengths(params)), len(params), step, C.addressof(config))
+
+    @staticmethod
+    def _check_lists(op, validator, lists):
+        """What `op` asks of its operands, of every entry of lists that run its f32 kernel side by side."""
+        if len({len(ts) for ts in lists}) != 1:
+            raise OjasError(SHAPE, f"{op}: lists of different lengths")
+        # Lists of matrices that fit, in one pass; the validator takes the others and says what is wrong.
+        every = [t for ts in lists for t in ts]
+        if {type(t) for t in every} == {DeviceTensor} and {(t.dtype, len(t.shape)) for t in every} == {(F32, 2)}:
+            dims = [t.shape for t in lists[0]]
+            if all([t.shape for t in ts] == dims for ts in lists[1:]) and all([t.numel for t in every]):
+                return
+        for entry in zip(*lists):
+            try:
+                validator(*entry)
+            except shapes.ShapeError as e:
+                raise OjasError(e.code, f"{e.op}: {e.detail}") from None
+        for t in every:
+            if not isinstance(t, DeviceTensor):
+                raise OjasError(PLACEMENT, f"{op}: operand is in host memory")
+            if t.dtype != F32:
+                raise OjasError(DTYPE, f"{op}: an f32 tensor is expected")
 
     @staticmethod
     def _pointers(ts):
@@ -586,6 +605,7 @@ class MiBackend(_native.Methods):
     def muon_ns5_step_list(self, params, grads, momenta, config: MuonNs5Config, params_bf16=None):
         """The same, each tensor all-or-nothing by itself, within 256 MiB of scratch and whatever less the budget has
         room for."""
+        self._check_lists("muon_ns5_step", shapes.muon_ns5_step_dims, (params, grads, momenta))
         self._muon_list(_native.omx_muon_ns5_step_list, params, grads, momenta, config, params_bf16)
 
     def _muon_list(self, entry, params, grads, momenta, config, params_bf16):
@@ -614,18 +634,24 @@ class MiBackend(_native.Methods):
         _native.omx_residual_add(self._context, x, x.dtype, y, y.dtype, out, od, x.numel)
         return out
 
+    @staticmethod
+    def _f32(op, *tensors):
+        if any(t.dtype != F32 for t in tensors):  # the kernel reads and writes four bytes an element
+            raise OjasError(DTYPE, f"{op}: an f32 tensor is expected")
+
     def accumulate_grad(self, acc, grad):
+        self._f32("accumulate_grad", acc, grad)
         _native.omx_accumulate_grad(self._context, acc, grad, acc.numel)
 
     def accumulate_grads(self, accs, grads):
         """`accumulate_grad` on several pairs in one launch."""
-        if len(accs) != len(grads) or any(a.numel != g.numel for a, g in zip(accs, grads)):
-            raise OjasError(SHAPE, "accumulate_grads: one gradient of the same size for each accumulator")
+        self._check_lists("accumulate_grad", lambda acc, grad: shapes.elementwise_dims("accumulate_grad", acc, grad), (accs, grads))
         tables = self._pointers(accs), self._pointers(grads)
         _native.omx_accumulate_grads(self._context, *[C.addressof(t) for t in tables],
                                      C.addressof(lens := self._lengths(accs)), len(accs))
 
     def scale_grad(self, grad, scale: float):
+        self._f32("scale_grad", grad)
         _native.omx_scale_grad(self._context, grad, scale, grad.numel)
 
     def _gelu(self, x, tanh_form):

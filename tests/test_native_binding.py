@@ -52,3 +52,52 @@ def test_native_methods_leave_what_does_not_fit_to_the_python_ones():
                  lambda: be.linear_forward(dev(2, 3), dev(4, 3), None, 1), lambda: be.linear_forward(dev(2, 3), dev(4, 3), x=1)):
         with pytest.raises(TypeError):
             call()
+
+
+@pytest.mark.parametrize("method", ["accumulate_grads", "muon_ns5_step_list", "adamw_step_batched"])
+def test_lists_are_checked_as_each_of_their_entries_is(method):
+    """A list op refuses what the op on one entry refuses, with its error: shapes (not sizes alone), dtypes, placement."""
+    from ojas_amd.backend import DTYPE, PLACEMENT, U32, AdamWConfig, MiBackend, MuonNs5Config
+
+    be = MiBackend.__new__(MiBackend)  # no device: nothing here gets as far as the library
+    be._ctx, be._context = None, _native.Context(0)
+
+    def dev(*shape, dtype=F32):
+        return DeviceTensor(be, 4096, shape, dtype, owns=False)
+
+    width = {"accumulate_grads": 2, "muon_ns5_step_list": 3, "adamw_step_batched": 4}[method]
+    extra = {"accumulate_grads": (), "muon_ns5_step_list": (MuonNs5Config.nanolab_default(),),
+             "adamw_step_batched": (0, AdamWConfig.nanolab(1e-3, 0.1))}[method]
+    good = lambda: [[dev(4, 6) for _ in range(3)] for _ in range(width)]
+    host = np.zeros((4, 6), np.float32)
+    for code, bad in [(SHAPE, dev(6, 4)), (SHAPE, dev(24)), (DTYPE, dev(4, 6, dtype=U32)), (DTYPE, dev(4, 6, dtype=BF16)), (PLACEMENT, host)]:
+        for which in range(1, width):
+            lists = good()
+            lists[which][2] = bad
+            with pytest.raises(OjasError) as e:
+                getattr(be, method)(*lists, *extra)
+            assert e.value.code == code, (which, e.value)
+    short = good()
+    short[-1].pop()
+    with pytest.raises(OjasError) as e:
+        getattr(be, method)(*short, *extra)
+    assert e.value.code == SHAPE
+    empty = good()
+    for ts in empty:
+        ts[1] = dev(0, 6)
+    with pytest.raises(OjasError) as e:
+        getattr(be, method)(*empty, *extra)
+    assert e.value.code == SHAPE
+
+
+def test_ops_that_know_f32_alone_refuse_other_storage():
+    from ojas_amd.backend import DTYPE, MiBackend
+
+    be = MiBackend.__new__(MiBackend)
+    be._ctx, be._context = None, _native.Context(0)
+    dev = lambda dtype: DeviceTensor(be, 4096, (8,), dtype, owns=False)
+    for call in (lambda: be.scale_grad(dev(BF16), 0.5), lambda: be.accumulate_grad(dev(BF16), dev(BF16)),
+                 lambda: be.accumulate_grad(dev(F32), dev(BF16))):
+        with pytest.raises(OjasError) as e:
+            call()
+        assert e.value.code == DTYPE
