@@ -21,9 +21,24 @@ import numpy as np
 from . import shapes
 try:
     from . import _native
+    from ._native import DeviceTensor  # a contiguous device tensor (host/py_native.cpp)
 except ImportError as _e:
-    raise ImportError("ojas_amd/_native.so is not built; run __graft_entry__.build()") from _e
-from ._native import DeviceTensor  # a contiguous device tensor (host/py_native.cpp)
+    _WHY = f"ojas_amd/_native.so is not built; run __graft_entry__.build() ({_e})"
+
+    class _Unbuilt:
+        """In the place of `_native`: the module's names, constants and validators can be had without it, no call can."""
+
+        class Methods:
+            pass
+
+        def __getattr__(self, name):
+            raise OjasError(BACKEND, _WHY)
+
+    class DeviceTensor:
+        def __init__(self, *_args, **_kwargs):
+            raise OjasError(BACKEND, _WHY)
+
+    _native = _Unbuilt()
 
 LIB_PATH = Path(__file__).resolve().parent / "libojas_mi355x.so"
 

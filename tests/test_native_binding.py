@@ -101,3 +101,33 @@ def test_ops_that_know_f32_alone_refuse_other_storage():
         with pytest.raises(OjasError) as e:
             call()
         assert e.value.code == DTYPE
+
+
+def test_the_package_imports_without_anything_built(tmp_path):
+    """Names, constants, configurations and validators need no library; a backend or a tensor says what is missing."""
+    import shutil
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    package = Path(_native.__file__).resolve().parent
+    (tmp_path / "ojas_amd").mkdir()
+    for source in package.glob("*.py"):
+        shutil.copy(source, tmp_path / "ojas_amd")
+    program = """
+import numpy as np
+import ojas_amd, ojas_amd.autocast, ojas_amd.lora, ojas_amd.nanolab, ojas_amd.trainer
+from ojas_amd import shapes
+from ojas_amd.backend import BACKEND, F32, AdamWConfig, DeviceTensor, MiBackend, OjasError
+assert shapes.linear_forward_dims(np.zeros((2, 4), np.float32), np.zeros((5, 4), np.float32))[0] == 2
+assert AdamWConfig.nanolab(1e-3, 0.1).beta2 == 0.95
+for make in (MiBackend, lambda: DeviceTensor(None, 0, (2, 3), F32)):
+    try:
+        make()
+    except OjasError as e:
+        assert e.code == BACKEND and "is not built" in e.detail, e
+    else:
+        raise AssertionError(make)
+"""
+    done = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
