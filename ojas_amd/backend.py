@@ -1043,7 +1043,7 @@ def _shape_first(name, method, validator, operands):
         except shapes.ShapeError as e:
             raise OjasError(e.code, f"{e.op}: {e.detail}") from None
         for t in args[:operands]:
-            if type(t) is not DeviceTensor and t is not None:
+            if not isinstance(t, DeviceTensor) and t is not None:
                 raise OjasError(PLACEMENT, f"{name}: operand is in host memory")
         return method(self, *args, **kwargs)
 

@@ -79,6 +79,8 @@ struct Tensor {
   PyObject* backend;  // the MiBackend (None once dropped)
   PyObject* shape;    // tuple of int
   PyObject* base;     // the tensor a view keeps alive
+  PyObject* dict;     // attributes a caller gives it (null until one does)
+  PyObject* weak;     // weak references to it
   unsigned long long ptr;
   Py_ssize_t numel;
   int dtype;
@@ -140,36 +142,67 @@ Tensor* make_tensor(PyObject* backend, Context* context, unsigned long long ptr,
   return t;
 }
 
+// The context of a backend, or null (a new reference).
+Context* context_in(PyObject* backend) {
+  PyObject* context = backend == Py_None ? nullptr : PyObject_GetAttrString(backend, "_context");
+  if (!context) PyErr_Clear();
+  if (context && Py_TYPE(context) != &ContextType) Py_CLEAR(context);
+  return reinterpret_cast<Context*>(context);
+}
+// A tensor of no elements and no memory until its __init__ (a subclass may have one of its own).
+PyObject* tensor_new(PyTypeObject* type, PyObject*, PyObject*) {
+  PyObject* shape = PyTuple_New(0);
+  if (!shape) return nullptr;
+  Tensor* t = reinterpret_cast<Tensor*>(type->tp_alloc(type, 0));
+  if (!t) {
+    Py_DECREF(shape);
+    return nullptr;
+  }
+  Py_INCREF(Py_None);
+  t->backend = Py_None;
+  t->shape = shape;
+  t->numel = 1;
+  return reinterpret_cast<PyObject*>(t);
+}
 // DeviceTensor(backend, ptr, shape, dtype, owns=True)
-PyObject* tensor_new(PyTypeObject*, PyObject* args, PyObject* kwargs) {
+int tensor_init(PyObject* self, PyObject* args, PyObject* kwargs) {
   static const char* names[] = {"backend", "ptr", "shape", "dtype", "owns", nullptr};
   PyObject *backend, *ptr_obj, *given;
   int dtype, owns = 1;
   if (!PyArg_ParseTupleAndKeywords(args, kwargs, "OOOi|p", const_cast<char**>(names), &backend, &ptr_obj, &given, &dtype, &owns))
-    return nullptr;
+    return -1;
   unsigned long long ptr = 0;
   if (ptr_obj != Py_None) {
     ptr = PyLong_AsUnsignedLongLong(ptr_obj);
-    if (PyErr_Occurred()) return nullptr;
+    if (PyErr_Occurred()) return -1;
   }
-  PyObject* context = backend == Py_None ? nullptr : PyObject_GetAttrString(backend, "_context");
-  if (!context) PyErr_Clear();
-  if (context && Py_TYPE(context) != &ContextType) Py_CLEAR(context);
   PyObject* shape = shape_tuple(given);
-  if (!shape) {
-    Py_XDECREF(context);
-    return nullptr;
-  }
+  if (!shape) return -1;
   const Py_ssize_t n = elements(shape);
-  Tensor* t = n == -1 && PyErr_Occurred() ? nullptr
-                                          : make_tensor(backend, reinterpret_cast<Context*>(context), ptr, shape, n, dtype, owns);
-  Py_XDECREF(context);
-  return reinterpret_cast<PyObject*>(t);
+  if (n == -1 && PyErr_Occurred()) {
+    Py_DECREF(shape);
+    return -1;
+  }
+  Tensor* t = reinterpret_cast<Tensor*>(self);
+  PyObject *old_backend = t->backend, *old_shape = t->shape, *old_context = reinterpret_cast<PyObject*>(t->context);
+  Py_INCREF(backend);
+  t->backend = backend;
+  t->context = context_in(backend);
+  t->shape = shape;
+  t->ptr = ptr;
+  t->numel = n;
+  t->dtype = dtype;
+  t->owns = owns;
+  Py_XDECREF(old_backend);
+  Py_XDECREF(old_shape);
+  Py_XDECREF(old_context);
+  return 0;
 }
 
 void tensor_dealloc(PyObject* self) {
   Tensor* t = reinterpret_cast<Tensor*>(self);
   PyObject_GC_UnTrack(self);
+  if (t->weak) PyObject_ClearWeakRefs(self);
   if (t->owns && t->ptr && t->context && t->context->ctx && p_free) {
     // A block too large for the context's pool goes back to the driver, which waits for the stream.
     PyThreadState* unlocked = t->numel >= (64l << 20) ? PyEval_SaveThread() : nullptr;
@@ -180,21 +213,48 @@ void tensor_dealloc(PyObject* self) {
   Py_XDECREF(t->backend);
   Py_XDECREF(t->shape);
   Py_XDECREF(t->base);
+  Py_XDECREF(t->dict);
   Py_TYPE(self)->tp_free(self);
 }
 int tensor_traverse(PyObject* self, visitproc visit, void* arg) {
   Tensor* t = reinterpret_cast<Tensor*>(self);
   Py_VISIT(t->backend);
   Py_VISIT(t->base);
+  Py_VISIT(t->dict);
   return 0;
 }
 int tensor_clear(PyObject* self) {
   Tensor* t = reinterpret_cast<Tensor*>(self);
   Py_CLEAR(t->base);
+  Py_CLEAR(t->dict);
   PyObject* backend = t->backend;
   Py_INCREF(Py_None);
   t->backend = Py_None;
   Py_XDECREF(backend);
+  return 0;
+}
+
+PyObject* tensor_shape(PyObject* self, void*) {
+  PyObject* shape = reinterpret_cast<Tensor*>(self)->shape;
+  Py_INCREF(shape);
+  return shape;
+}
+int tensor_set_shape(PyObject* self, PyObject* given, void*) {
+  Tensor* t = reinterpret_cast<Tensor*>(self);
+  PyObject* shape = given ? shape_tuple(given) : nullptr;
+  if (!shape) {
+    if (!given) PyErr_SetString(PyExc_AttributeError, "shape");
+    return -1;
+  }
+  const Py_ssize_t n = elements(shape);
+  if (n == -1 && PyErr_Occurred()) {
+    Py_DECREF(shape);
+    return -1;
+  }
+  t->numel = n;
+  PyObject* old = t->shape;
+  t->shape = shape;
+  Py_DECREF(old);
   return 0;
 }
 
@@ -233,9 +293,8 @@ PyMethodDef tensor_methods[] = {{"reshape", tensor_reshape, METH_VARARGS, "A zer
                                 {nullptr, nullptr, 0, nullptr}};
 PyMemberDef tensor_members[] = {
     {"backend", T_OBJECT, offsetof(Tensor, backend), READONLY, nullptr},
-    {"shape", T_OBJECT, offsetof(Tensor, shape), READONLY, nullptr},
     {"ptr", T_ULONGLONG, offsetof(Tensor, ptr), 0, nullptr},
-    {"dtype", T_INT, offsetof(Tensor, dtype), READONLY, nullptr},
+    {"dtype", T_INT, offsetof(Tensor, dtype), 0, nullptr},
     {"numel", T_PYSSIZET, offsetof(Tensor, numel), READONLY, nullptr},
     {"_owns", T_BOOL, offsetof(Tensor, owns), 0, nullptr},
     {"_base", T_OBJECT, offsetof(Tensor, base), READONLY, nullptr},
@@ -243,7 +302,9 @@ PyMemberDef tensor_members[] = {
     // to be bf16-exact, so a second rounding would only clone. Set by `Autocast`.
     {"compute_bf16", T_BOOL, offsetof(Tensor, compute_bf16), 0, nullptr},
     {nullptr, 0, 0, 0, nullptr}};
-PyGetSetDef tensor_getset[] = {{"nbytes", tensor_nbytes, nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyGetSetDef tensor_getset[] = {{"shape", tensor_shape, tensor_set_shape, nullptr, nullptr},
+                               {"__dict__", PyObject_GenericGetDict, PyObject_GenericSetDict, nullptr, nullptr},
+                               {"nbytes", tensor_nbytes, nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
 
 // empty(backend, context, shape, dtype): a new tensor charged to the context's budget.
 PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -289,7 +350,7 @@ bool convert(PyObject* o, T* out) {
     *out = reinterpret_cast<Context*>(o)->ctx;
     return true;
   } else if constexpr (std::is_pointer_v<T>) {
-    if (Py_TYPE(o) == &TensorType) {
+    if (PyObject_TypeCheck(o, &TensorType)) {
       *out = reinterpret_cast<T>(reinterpret_cast<Tensor*>(o)->ptr);
       return true;
     }
@@ -429,7 +490,7 @@ bool bind(PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames, const char
   return true;
 }
 
-const Tensor* tensor_in(PyObject* o) { return o && Py_TYPE(o) == &TensorType ? reinterpret_cast<const Tensor*>(o) : nullptr; }
+const Tensor* tensor_in(PyObject* o) { return o && PyObject_TypeCheck(o, &TensorType) ? reinterpret_cast<const Tensor*>(o) : nullptr; }
 // A float tensor with elements, as the validators ask of every operand.
 const Tensor* floats_in(PyObject* o) {
   const Tensor* t = tensor_in(o);
@@ -723,8 +784,11 @@ PyMODINIT_FUNC PyInit__native(void) {
       "A contiguous device tensor: pointer, shape, dtype. Frees itself on drop\n"
       "(the role of `Arc<dyn DeviceBuffer>` + `Reservation`, tensor.rs:146-163).";
   TensorType.tp_basicsize = sizeof(Tensor);
-  TensorType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  TensorType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC | Py_TPFLAGS_BASETYPE;
+  TensorType.tp_dictoffset = offsetof(Tensor, dict);
+  TensorType.tp_weaklistoffset = offsetof(Tensor, weak);
   TensorType.tp_new = tensor_new;
+  TensorType.tp_init = tensor_init;
   TensorType.tp_dealloc = tensor_dealloc;
   TensorType.tp_traverse = tensor_traverse;
   TensorType.tp_clear = tensor_clear;

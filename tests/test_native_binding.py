@@ -131,3 +131,67 @@ for make in (MiBackend, lambda: DeviceTensor(None, 0, (2, 3), F32)):
 """
     done = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True)
     assert done.returncode == 0, done.stderr
+
+
+class Named(DeviceTensor):
+    def __init__(self, name, *args, **kwargs):
+        super().__init__(*args, **kwargs)
+        self.name = name
+
+
+def test_a_tensor_is_an_ordinary_python_object():
+    """Attributes, subclasses with an __init__ of their own, weak references, a shape and a dtype that can be set."""
+    import gc
+    import weakref
+
+    from ojas_amd.backend import MiBackend
+
+    t = DeviceTensor(None, 4096, (2, 3), F32, owns=False)
+    t.label, t.me = "weights", t  # a cycle
+    assert t.label == "weights" and t.__dict__["me"] is t
+    gone = []
+    ref = weakref.ref(t, gone.append)
+    assert ref() is t
+    del t
+    gc.collect()
+    assert ref() is None and gone == [ref]
+    s = Named("q", None, 4096, [4, 6], BF16, owns=False)
+    assert isinstance(s, DeviceTensor) and (s.name, s.shape, s.numel, s.nbytes) == ("q", (4, 6), 24, 48)
+    assert weakref.ref(s)() is s and s.reshape(24).shape == (24,)
+    s.shape, s.dtype = [3, 4], F32
+    assert (s.shape, s.numel, s.nbytes) == ((3, 4), 12, 48)
+    with pytest.raises(AttributeError):
+        s.nothing
+    with pytest.raises(TypeError):
+        DeviceTensor(None, 0, (2,))
+    # Operands of a subclass pass for tensors: what is wrong with this call is its shapes.
+    be = MiBackend.__new__(MiBackend)
+    be._ctx, be._context = None, _native.Context(0)
+    for call in (lambda: be.linear_forward(Named("x", be, 4096, (2, 3), F32, owns=False), Named("w", be, 4096, (4, 5), F32, owns=False)),
+                 lambda: be.accumulate_grads([Named("a", be, 4096, (2,), F32, owns=False)], [Named("g", be, 4096, (3,), F32, owns=False)])):
+        with pytest.raises(OjasError) as e:
+            call()
+        assert e.value.code == SHAPE
+
+
+@pytest.mark.gpu
+def test_a_subclass_owns_its_memory_as_a_tensor_does():
+    import gc
+
+    from ojas_amd.backend import MiBackend
+
+    be = MiBackend(0)
+    live = be.budget()["live"]
+    t = be.empty((1024,))
+    t._owns = False  # handed over
+    s = Named("moved", be, t.ptr, t.shape, t.dtype)
+    del t
+    assert be.budget()["live"] == live + 4096
+    x = np.arange(1024, dtype=np.float32)
+    _native.omx_upload(be._context, s, 0, x.ctypes.data, x.nbytes)
+    assert np.array_equal(be.download(be.residual_add_forward(s, s)), x + x)
+    s.me = s
+    del s
+    gc.collect()
+    assert be.budget()["live"] == live
+    be.close()
