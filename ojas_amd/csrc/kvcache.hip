@@ -519,7 +519,7 @@ __global__ __launch_bounds__(64) void cached_attention_merge_kernel(KvArgs a, lo
 struct KvWrite {
   void* cache;
   const float* src;
-  unsigned int* refused;  // of the two-launch form: holds the tag of the last scan that refused
+  unsigned int* refused;  // of the two-launch form: 64 bits with the tag of a scan that refused, then how many workgroups saw it
   size_t n;               // elements of src
   unsigned int capacity, step, tn, at;  // at: already modulo the capacity
   OmxFaultWord* fault;
@@ -593,7 +593,8 @@ __global__ __launch_bounds__(KV_SCAN_THREADS) void kv_scan_write_kernel(KvWrite 
   }
 }
 // A longer one: the first launch scans, the second copies unless the scan refused. The word between them
-// holds the tag of a refused scan, which no other call shares, so nothing has to be cleared.
+// holds the tag of a refused scan; the second launch's last workgroup takes it back, for a replay of the two out of a
+// captured graph comes with the same tag (nothing is cleared where nothing was refused).
 template <int VEC>
 __global__ __launch_bounds__(256) void kv_scan_kernel(KvWrite w) {
   bool bad = false;
@@ -606,7 +607,14 @@ __global__ __launch_bounds__(256) void kv_scan_kernel(KvWrite w) {
 }
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void kv_write_kernel(KvWrite w) {
-  if (*reinterpret_cast<const unsigned long long*>(w.refused) == w.tag) return;
+  if (*reinterpret_cast<const volatile unsigned long long*>(w.refused) == w.tag) {
+    __syncthreads();  // the whole workgroup has read it
+    if (threadIdx.x == 0 && atomicAdd(w.refused + 2, 1u) == gridDim.x - 1) {
+      w.refused[2] = 0u;
+      atomicExch(reinterpret_cast<unsigned long long*>(w.refused), 0ull);
+    }
+    return;
+  }
   for (size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * VEC; i < w.n; i += static_cast<size_t>(gridDim.x) * 256 * VEC)
     kv_put<T, VEC>(w, i);
 }

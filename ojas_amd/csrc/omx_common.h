@@ -77,7 +77,7 @@ struct omx_ctx {
   uint64_t pooled_bytes = 0;
   OmxFaultWord* fault = nullptr;  // device
   OmxFaultWord* fault_host = nullptr;  // pinned
-  unsigned int* kv_refused = nullptr;  // device, behind the fault word: the tag of the last refused cache write (64 bits)
+  unsigned int* kv_refused = nullptr;  // device, behind the fault word: KvWrite::refused, zero between calls
   uint64_t sequence = 0;
   std::string last_error;
   std::string arch;

@@ -313,3 +313,41 @@ def test_few_rows_over_a_long_cache_are_no_slower_than_a_wave_per_four_rows(be):
             be.sync()
             best = min(best, (time.perf_counter() - start) / 20)
         assert best <= 50e-6, best
+
+
+def test_a_replayed_cache_write_forgets_a_refusal(be):
+    """The two-launch write out of a captured graph: a replay whose source is not finite writes nothing, and the next one, the
+    same launches with the same arguments, writes again."""
+    import ctypes as C
+
+    print("kv cache write, replayed", flush=True)
+    hip, stream = be._lib, C.c_void_p(be.stream())
+    r = np.random.default_rng(3)
+    shape = (2, 24, 8, 64)  # 24576 values
+    cache, src = be.zeros(shape), be.zeros(shape)
+    be.kv_cache_write(cache, src, 0)
+    be.sync()
+    graph, program = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, C.c_int(2)) == 0
+    be.kv_cache_write(cache, src, 0)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(program), graph, None, None, C.c_size_t(0)) == 0
+
+    def load(values):
+        be._check(be._lib.omx_upload(be._ctx, be._p(src), C.c_uint64(0), values.ctypes.data_as(C.c_void_p), C.c_uint64(values.nbytes)))
+
+    before = be.download(cache)
+    for step in range(6):
+        values = r.standard_normal(shape).astype(np.float32)
+        if step % 3 == 1:
+            values[-1, -1, -1, -1] = np.nan
+        load(values)
+        assert hip.hipGraphLaunch(program, stream) == 0
+        if step % 3 == 1:
+            with pytest.raises(OjasError):
+                be.sync()
+        else:
+            before = values
+        assert np.array_equal(be.download(cache), before), step
+    hip.hipGraphExecDestroy(program)
+    hip.hipGraphDestroy(graph)
