@@ -415,31 +415,31 @@ int dma_splits(long tiles, int ksteps) {
 // steps, the steps, the store pass by output elements, and a split's second launch with its partial sums (8 bytes per
 // element and split, out of the caches). A step takes `one` with at most one tile per compute unit and `more` for each
 // tile of the fullest unit beyond that: its tiles share the LDS, so each waits for less. (256 x 128 tiles, whose eight
-// waves start the next tile while others finish, go by the mean instead.) An output whose rows are not 16-byte aligned is
-// stored value by value, a tile's worth per round.
-// Fitted by least squares to 2500 timings: 256 .. 8192 rows, 333 .. 3072 columns, K = 512 .. 16384 split 1 to 16
-// ways, all layouts: 8 % rms. What it picks is 1 % behind the fastest on average (weight gradients of 1024 x 1024 over
-// 8192 / 16384 tokens: 34.1 / 55.9 -> 29.9 / 44.2 us, of 768 x 768 over 4096: 24.7 -> 16.0, against one step time for
-// every number of tiles on a unit and a larger tiling judged at one split only).
+// waves start the next tile while others finish, go halfway between the fullest unit and the mean.) An activation's store
+// pass, and one value by value into an output whose rows are not 16-byte aligned, count a tile at a time.
+// Fitted by least squares to 3500 timings: 256 .. 16384 rows, 333 .. 5504 columns, K = 128 .. 16384 split 1 to 16
+// ways, all layouts, with and without an activation: 8 % rms. What it picks is 1.1 % behind the fastest on average
+// (weight gradients of 1024 x 1024 over 8192 / 16384 tokens: 34.1 / 55.9 -> 29.9 / 44.2 us, of 768 x 768 over 4096:
+// 24.7 -> 16.0, against one step time for every number of tiles on a unit and a larger tiling judged at one split only).
 double dma_us(int variant, long m, long n, long batches, int ksteps, int splits, bool a_km, bool activation, bool unaligned,
               long cus) {
   struct Cost {
     double base, activation, unaligned, one[2], more[2];  // [k-contiguous A, k-major A]
   };
-  static constexpr Cost kCosts[4] = {{3.5, 2.8, 7.5, {0.70, 0.64}, {0.86, 0.80}},    // 3: 256 x 128
-                                     {3.0, 1.5, 8.0, {0.51, 0.53}, {0.44, 0.39}},    // 6: 128 x 128
-                                     {3.4, 0.9, 2.2, {0.32, 0.35}, {0.245, 0.27}},   // 7: 128 x 64
-                                     {2.7, 0.7, 1.6, {0.20, 0.21}, {0.17, 0.18}}};   // 8: 64 x 64
+  static constexpr Cost kCosts[4] = {{3.9, 3.2, 7.5, {0.71, 0.64}, {0.82, 0.77}},      // 3: 256 x 128
+                                     {3.4, 1.6, 8.0, {0.55, 0.53}, {0.46, 0.395}},     // 6: 128 x 128
+                                     {3.4, 0.9, 2.2, {0.32, 0.355}, {0.245, 0.275}},   // 7: 128 x 64
+                                     {2.9, 0.35, 1.6, {0.197, 0.21}, {0.167, 0.18}}};  // 8: 64 x 64
   const Cost& c = kCosts[variant == 3 ? 0 : variant - 5];
   int bm, bn;
   omx_gemm_dma_tile(variant, &bm, &bn);
   const long groups = ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batches * splits;
-  const double fullest = variant == 3 ? static_cast<double>(groups) / static_cast<double>(cus)
-                                      : static_cast<double>((groups + cus - 1) / cus);
-  const double step = groups <= cus ? c.one[a_km] : std::max(c.one[a_km], c.more[a_km] * fullest);
+  const double fullest = static_cast<double>((groups + cus - 1) / cus), mean = static_cast<double>(groups) / static_cast<double>(cus);
+  const double tiles = variant == 3 ? std::max(1.0, 0.5 * (fullest + mean)) : fullest;
+  const double step = groups <= cus ? c.one[a_km] : std::max(c.one[a_km], c.more[a_km] * tiles);
   const double out = 1e-6 * static_cast<double>(m) * static_cast<double>(n) * static_cast<double>(batches);
-  return c.base + (activation ? c.activation : 0.0) + (unaligned ? c.unaligned * std::max(1.0, fullest) : 0.0) +
-         step * ((ksteps + splits - 1) / splits) + 0.7 * out + (splits > 1 ? 5.8 + 0.17 * splits + 1.05 * out * splits : 0.0);
+  return c.base + tiles * ((activation ? c.activation : 0.0) + (unaligned ? c.unaligned : 0.0)) +
+         step * ((ksteps + splits - 1) / splits) + 0.48 * out + (splits > 1 ? 5.7 + 0.17 * splits + 1.07 * out * splits : 0.0);
 }
 
 // The cheapest split of a product over such a tiling, at most `limit` ways.
