@@ -579,22 +579,20 @@ class MiBackend(_native.Methods):
                                        C.addressof(lens := self._lengths(params)), len(params), step, C.addressof(config))
 
     @staticmethod
-    def _check_lists(op, validator, lists):
+    def _check_lists(op, validator, lists, rank=None):
         """What `op` asks of its operands, of every entry of lists that run its f32 kernel side by side."""
         if len({len(ts) for ts in lists}) != 1:
             raise OjasError(SHAPE, f"{op}: lists of different lengths")
-        # Lists of matrices that fit, in one pass; the validator takes the others and says what is wrong.
-        every = [t for ts in lists for t in ts]
-        if {type(t) for t in every} == {DeviceTensor} and {(t.dtype, len(t.shape)) for t in every} == {(F32, 2)}:
-            dims = [t.shape for t in lists[0]]
-            if all([t.shape for t in ts] == dims for ts in lists[1:]) and all([t.numel for t in every]):
-                return
+        # Well-formed lists in one pass; the validator says what is wrong with others.
+        match = _native.lists_match(*lists)
+        if match >= 0 and rank in (None, match):
+            return
         for entry in zip(*lists):
             try:
                 validator(*entry)
             except shapes.ShapeError as e:
                 raise OjasError(e.code, f"{e.op}: {e.detail}") from None
-        for t in every:
+        for t in (t for ts in lists for t in ts):
             if not isinstance(t, DeviceTensor):
                 raise OjasError(PLACEMENT, f"{op}: operand is in host memory")
             if t.dtype != F32:
@@ -620,7 +618,7 @@ class MiBackend(_native.Methods):
     def muon_ns5_step_list(self, params, grads, momenta, config: MuonNs5Config, params_bf16=None):
         """The same, each tensor all-or-nothing by itself, within 256 MiB of scratch and whatever less the budget has
         room for."""
-        self._check_lists("muon_ns5_step", shapes.muon_ns5_step_dims, (params, grads, momenta))
+        self._check_lists("muon_ns5_step", shapes.muon_ns5_step_dims, (params, grads, momenta), rank=2)
         self._muon_list(_native.omx_muon_ns5_step_list, params, grads, momenta, config, params_bf16)
 
     def _muon_list(self, entry, params, grads, momenta, config, params_bf16):

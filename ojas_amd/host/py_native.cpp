@@ -337,6 +337,31 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return reinterpret_cast<PyObject*>(t);
 }
 
+// lists_match(list, list, ...), of one length: whether every entry's tensors are f32, have elements and share a shape. Returns
+// their rank (0 where entries differ in it), or -1.
+PyObject* lists_match(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs < 1) return PyLong_FromLong(-1);
+  Py_ssize_t rank = -1;
+  for (Py_ssize_t l = 0; l < nargs; ++l)
+    if (!PyList_CheckExact(args[l]) || PyList_GET_SIZE(args[l]) != PyList_GET_SIZE(args[0])) return PyLong_FromLong(-1);
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); ++i) {
+    PyObject* first = nullptr;
+    for (Py_ssize_t l = 0; l < nargs; ++l) {
+      PyObject* o = PyList_GET_ITEM(args[l], i);
+      if (Py_TYPE(o) != &TensorType) return PyLong_FromLong(-1);
+      const Tensor* t = reinterpret_cast<const Tensor*>(o);
+      if (t->dtype != 0 || t->numel <= 0) return PyLong_FromLong(-1);
+      if (!first) first = t->shape;
+      const int same = first == t->shape ? 1 : PyObject_RichCompareBool(first, t->shape, Py_EQ);
+      if (same < 0) return nullptr;
+      if (!same) return PyLong_FromLong(-1);
+    }
+    const Py_ssize_t own = PyTuple_GET_SIZE(first);
+    rank = rank == -1 || rank == own ? own : 0;
+  }
+  return PyLong_FromSsize_t(rank);
+}
+
 // ---- typed calls ----
 // One argument converted into parameter type T. A pointer is a tensor's memory, null or a plain
 // address; a host array is refused (its address would reach a kernel).
@@ -765,6 +790,7 @@ PyObject* load(PyObject*, PyObject* args) {
   {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Entry<ID_##name, decltype(::name)>::call)), METH_FASTCALL, nullptr},
 PyMethodDef module_methods[] = {
     OMX_ENTRIES(X){"load", load, METH_VARARGS, "load(path, error_type)"},
+    {"lists_match", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&lists_match)), METH_FASTCALL, "lists_match(list, ...)"},
     {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&empty)), METH_FASTCALL, "empty(backend, context, shape, dtype)"},
     {nullptr, nullptr, 0, nullptr}};
 #undef X
