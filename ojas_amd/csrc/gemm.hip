@@ -415,31 +415,35 @@ int dma_splits(long tiles, int ksteps) {
 // steps, the steps, the store pass by output elements, and a split's second launch with its partial sums (8 bytes per
 // element and split, out of the caches). A step takes `one` with at most one tile per compute unit and `more` for each
 // tile of the fullest unit beyond that: its tiles share the LDS, so each waits for less. (256 x 128 tiles, whose eight
-// waves start the next tile while others finish, go halfway between the fullest unit and the mean.) An activation's store
-// pass, and one value by value into an output whose rows are not 16-byte aligned, count a tile at a time.
-// Fitted by least squares to 3500 timings: 256 .. 16384 rows, 333 .. 5504 columns, K = 128 .. 16384 split 1 to 16
-// ways, all layouts, with and without an activation: 8 % rms. What it picks is 1.1 % behind the fastest on average
-// (weight gradients of 1024 x 1024 over 8192 / 16384 tokens: 34.1 / 55.9 -> 29.9 / 44.2 us, of 768 x 768 over 4096:
-// 24.7 -> 16.0, against one step time for every number of tiles on a unit and a larger tiling judged at one split only).
+// waves start the next tile while others finish, go halfway between the fullest unit and the mean.) Over 2048 columns of
+// K and more the operands leave the nearest cache, which costs the smaller tiles, with their larger share of loads, up to
+// `far` more of a step (128 x 128 ones, by the fit, a tenth less). An activation's store pass, and one value by value into an output whose rows are not 16-byte aligned, count
+// a tile at a time.
+// Fitted to 7400 timings: 256 .. 16384 rows, 128 .. 5504 columns, K = 128 .. 50304 split 1 to 16 ways, all layouts, with
+// and without an activation, batches of 3, 6 and 12 weight gradients. What it picks among these tilings is 2.4 % behind the
+// fastest on average over 710 products (weight gradients of 1024 x 1024 over 8192 / 16384 tokens: 34.1 / 55.9 -> 29.9 /
+// 44.2 us, of 768 x 768 over 4096: 24.7 -> 16.0); one step time for every number of tiles on a unit, and a larger tiling
+// judged at one split only, picked 6 % behind.
 double dma_us(int variant, long m, long n, long batches, int ksteps, int splits, bool a_km, bool activation, bool unaligned,
               long cus) {
   struct Cost {
-    double base, activation, unaligned, one[2], more[2];  // [k-contiguous A, k-major A]
+    double base, activation, unaligned, one[2], more[2], far;  // [k-contiguous A, k-major A]
   };
-  static constexpr Cost kCosts[4] = {{3.9, 3.2, 7.5, {0.71, 0.64}, {0.82, 0.77}},      // 3: 256 x 128
-                                     {3.4, 1.6, 8.0, {0.55, 0.53}, {0.46, 0.395}},     // 6: 128 x 128
-                                     {3.4, 0.9, 2.2, {0.32, 0.355}, {0.245, 0.275}},   // 7: 128 x 64
-                                     {2.9, 0.35, 1.6, {0.197, 0.21}, {0.167, 0.18}}};  // 8: 64 x 64
+  static constexpr Cost kCosts[4] = {{4.2, 3.2, 7.5, {0.83, 0.69}, {0.82, 0.705}, 0.11},        // 3: 256 x 128
+                                     {3.4, 1.6, 8.0, {0.63, 0.545}, {0.473, 0.382}, -0.1},      // 6: 128 x 128
+                                     {3.3, 0.9, 2.2, {0.357, 0.354}, {0.249, 0.267}, 0.18},     // 7: 128 x 64
+                                     {3.0, 0.35, 1.6, {0.199, 0.219}, {0.175, 0.18}, 0.28}};    // 8: 64 x 64
   const Cost& c = kCosts[variant == 3 ? 0 : variant - 5];
   int bm, bn;
   omx_gemm_dma_tile(variant, &bm, &bn);
   const long groups = ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batches * splits;
   const double fullest = static_cast<double>((groups + cus - 1) / cus), mean = static_cast<double>(groups) / static_cast<double>(cus);
   const double tiles = variant == 3 ? std::max(1.0, 0.5 * (fullest + mean)) : fullest;
-  const double step = groups <= cus ? c.one[a_km] : std::max(c.one[a_km], c.more[a_km] * tiles);
+  const double far = 1.0 + c.far * std::min(1.0, std::max(0.0, (ksteps - 32) / 224.0));
+  const double step = groups <= cus ? c.one[a_km] : std::max(c.one[a_km], c.more[a_km] * tiles * far);
   const double out = 1e-6 * static_cast<double>(m) * static_cast<double>(n) * static_cast<double>(batches);
   return c.base + tiles * ((activation ? c.activation : 0.0) + (unaligned ? c.unaligned : 0.0)) +
-         step * ((ksteps + splits - 1) / splits) + 0.48 * out + (splits > 1 ? 5.7 + 0.17 * splits + 1.07 * out * splits : 0.0);
+         step * ((ksteps + splits - 1) / splits) + 0.55 * out + (splits > 1 ? 4.6 + 0.25 * splits + 1.18 * out * splits : 0.0);
 }
 
 // The cheapest split of a product over such a tiling, at most `limit` ways.
