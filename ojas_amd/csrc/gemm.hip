@@ -577,7 +577,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       if (a_km && b_km && unbatched && ksteps64 >= 64 && tiles128 < cus) {
         dma_variant = 6;
       } else if (outputs * g.batches <= (1l << 20)) {
-        dma_variant = -1;  // a handful of tiles: the register-staged kernel, which splits K freely
+        dma_variant = -1;  // a handful of tiles: the estimate below picks among the smaller ones, K split freely
       } else if (a_km && b_km) {
         // Weight gradients (K = tokens). An unbatched product with a poor last round is cut by rows below.
         if (plain && ksteps64 >= 64 && all256 >= cus && (unbatched || all256 * 5 >= rounds256 * cus * 4)) dma_variant = 9;

@@ -3,17 +3,14 @@
 //
 // Same contract as gemm.hip (C[M,N] (+)= A.B, f32 accumulation, every operand
 // layout; reference: ojas-cpu/src/linalg.rs:69-210), different data movement:
-//   * 512 threads (8 waves); tile 256 x 128 (waves 4 x 2, each 64 x 64) or 256 x 256 (waves
-//     2 x 4, each 128 x 64; half the L2-to-LDS traffic per FLOP).
-//   * Variant 3, the default: K steps of 32 columns, three stages in 72 KiB and at most 128
-//     VGPRs, so two workgroups share a compute unit and one's output stores, first loads and
-//     barrier waits overlap the other's products. Its weakness: a k-contiguous operand row
+//   * Variant 3: 512 threads (8 waves), tile 256 x 128 (waves 4 x 2, each 64 x 64). K steps of 32 columns,
+//     three stages in 72 KiB and at most 128 VGPRs, so two workgroups share a compute unit and one's output
+//     stores, first loads and barrier waits overlap the other's products. Its weakness: a k-contiguous operand row
 //     contributes half a 128-byte cache line per step, each line is requested twice, far enough
 //     apart that the second request misses L1 again, and the load path then delivers 65 GB/s
 //     per compute unit instead of 107 GB/s (measured with the loads alone).
-//   * Variant 0 (256 x 256, two stages): K steps of 64 columns, whole cache lines, one workgroup per
-//     compute unit. Load latency (about 0.6 us) is then exposed; it wins on long reductions with
-//     large outputs only.
+//   * Variants 6, 7, 8: 256 threads (4 waves, 2 x 2), tiles 128 x 128 in 32-column steps, 128 x 64 and 64 x 64 in
+//     64-column ones (whole cache lines); three or two workgroups per compute unit. gemm.hip's dma_us says when.
 //   * operand tiles go from global memory straight into LDS: no staging
 //     registers and no LDS store instructions. A wave-wide load writes 64
 //     consecutive 16-byte slots, so the LDS tile is unpadded and bank conflicts

@@ -92,7 +92,7 @@ struct omx_ctx {
   // when the context is opened (the lookup is not stream work and may load the code object).
   void* ce_static_scratch = nullptr;
   // Optional per-launch timing of the GEMM kernel (benchmark only).
-  // 0: 128x128 kernel only; 1: choose by shape; 2 / 3: force the 256x256 / 256x128 direct-to-LDS kernel where eligible.
+  // 0: 128x128 register-staged kernel only; 1: choose by shape; others force a direct-to-LDS tiling (omx_set_option).
   int gemm_dma_mode = 1;
   int gemm_row_split = 1;    // 0: a product whose last round of 256 x 256 tiles is mostly empty is not cut by rows
   bool gemm_in_row_split = false;  // set while omx_gemm_impl runs the two halves of a cut product
