@@ -18,6 +18,15 @@ __device__ __forceinline__ void wait_loads(int groups) {
   }
 }
 
+// Workgroup -> tile so that the workgroups of one XCD (equal index modulo 8) take a contiguous run of the tiles, also
+// where the count is no multiple of 8: the first count % 8 XCDs have one more. 684 x 5504 over 2048 on 64 x 64 tiles,
+// 946 of them: 47.8 us in index order, where neighbours sit behind eight different L2s, 24.9 in this one; 802 products
+// of 40 .. 16384 rows 4.5 % less on average.
+__device__ inline int dma_eighth(int index, int count) {
+  const int xcd = index & 7;
+  return xcd * (count >> 3) + min(xcd, count & 7) + (index >> 3);
+}
+
 // EPI: the store pass (OMX_EPI_*). A kernel of its own per store pass keeps each one's code (a few KiB of
 // straight-line stores) and registers out of the others. TAIL: see StepBase.
 template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI, bool TAIL = false>
@@ -43,16 +52,15 @@ gemm_dma_kernel(GemmArgs g) {
   // are fetched into one or two L2s instead of all eight.
   const int total = g.tiles_m * g.tiles_n;
   int split = 0, id = blockIdx.x, product = blockIdx.y;
-  if (g.batches > 1 && g.splits == 1 && ((total * g.batches) & 7) == 0) {
-    const int linear = blockIdx.y * total + blockIdx.x;
-    const int r = (linear & 7) * ((total * g.batches) >> 3) + (linear >> 3);
+  if (g.batches > 1 && g.splits == 1) {
+    const int r = dma_eighth(blockIdx.y * total + blockIdx.x, total * g.batches);
     product = r / total;
     id = r - product * total;
   } else if (g.splits > 1) {
     split = blockIdx.x % g.splits;
     id = blockIdx.x / g.splits;
-  } else if (total % 8 == 0) {
-    id = (id & 7) * (total >> 3) + (id >> 3);
+  } else {
+    id = dma_eighth(id, total);
   }
   const int band = 4;
   const int tiles_per_band = band * g.tiles_n;

@@ -153,6 +153,46 @@ def test_long_weight_gradients_take_a_tiling_within_a_tenth_of_the_best(be, m, t
     assert chosen <= 1.10 * min(forced.values()), (chosen, forced)
 
 
+def test_tiles_that_do_not_divide_by_the_xcds_run_as_those_that_do(be):
+    """684 rows by 5504 columns over 2048 are 11 x 86 tiles of 64 x 64, two more than a multiple of 8; 5632 columns are 11 x 88.
+    An XCD takes a contiguous eighth of either, so the smaller product takes no longer (1.15 for the spread of two short
+    runs; in index order 47.8 against some 25 us), and the choice for it is within a tenth of the tilings forced."""
+    from ojas_amd.backend import BF16
+
+    m, k = 684, 2048
+    print("gemm tile order 684 x 2048 x 5504 / 5632", flush=True)
+    a, b, c = be.empty((m * k,), BF16), be.empty((k * 5632,), BF16), be.empty((m * 5632,), BF16)
+    for t, seed in ((a, 1), (b, 2)):
+        be._check(be._lib.omx_init_normal(be._ctx, be._p(t), C.c_int32(BF16), C.c_uint64(t.numel), C.c_uint64(seed),
+                                          C.c_float(0.05)))
+
+    def us(mode, n):
+        be.set_option("gemm_dma", mode)
+        best = float("inf")
+        for _ in range(3):
+            be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(1)))
+            for _ in range(10):
+                be._check(be._lib.omx_gemm(be._ctx, be._p(a), C.c_uint64(k), C.c_uint64(1), be._p(b), C.c_uint64(1), C.c_uint64(k),
+                                           C.c_int32(BF16), be._p(c), C.c_int32(BF16), C.c_uint64(m), C.c_uint64(k), C.c_uint64(n),
+                                           C.c_int32(0)))
+            ms = C.c_double()
+            be._check(be._lib.omx_profile_gemm_report(be._ctx, None, C.byref(ms), None))
+            be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(0)))
+            best = min(best, ms.value * 100)
+        return best
+
+    try:
+        us(1, 5504)  # clocks up
+        even, odd = us(8, 5632), us(8, 5504)
+        forced = {mode: us(mode, 5504) for mode in (3, 4, 7, 8)}
+        chosen = us(1, 5504)
+    finally:
+        be.set_option("gemm_dma", 1)
+    print("  us: 5632 columns %.1f, 5504 %.1f; chosen %.1f, forced %s" % (even, odd, chosen, forced), flush=True)
+    assert odd <= 1.15 * even, (odd, even)
+    assert chosen <= 1.10 * min(forced.values()), (chosen, forced)
+
+
 def test_a_mostly_empty_last_round_is_cut_by_rows(be):
     """65 x 16 tiles of 256 x 256 are four rounds of the 256 compute units and 16 tiles more: the
     first 64 tile rows keep the tiling, the last goes to a launch of its own. Checked against the
@@ -251,7 +291,7 @@ def test_unknown_option_is_refused(be):
 
 
 @pytest.mark.parametrize("mode", [0, 1, 3, 4, 9, 10])
-@pytest.mark.parametrize("layers", [3, 4])  # 4: a tile count divisible by 8, which takes the XCD-ordered mapping
+@pytest.mark.parametrize("layers", [3, 4])  # tile counts that divide by the 8 XCDs evenly (4) and that do not (3)
 @pytest.mark.parametrize("rows,kin,nout", [(1088, 136, 264), (2048, 768, 256), (2048, 200, 328)])
 def test_strided_batch_of_weight_gradients(be, mode, rows, kin, nout, layers):
     """`omx_gemm_strided_batch` as the step driver uses it: gw[l] = gy[l]^T x[l] for three stacked
