@@ -417,11 +417,11 @@ int dma_splits(long tiles, int ksteps) {
 // tile of the fullest unit beyond that: its tiles share the LDS, so each waits for less. (256 x 128 tiles, whose eight
 // waves start the next tile while others finish, go halfway between the fullest unit and the mean.) Over 2048 columns of
 // K and more the operands leave the nearest cache, which costs the smaller tiles, with their larger share of loads, up to
-// `far` more of a step (128 x 128 ones, by the fit, a tenth less). An activation's store pass, and one value by value into an output whose rows are not 16-byte aligned, count
-// a tile at a time.
+// `far` more of a step (128 x 128 ones, by the fit, a tenth less). An activation's store pass, and one value by value into
+// an output whose rows are not 16-byte aligned, count a tile at a time.
 // Fitted to 7400 timings: 256 .. 16384 rows, 128 .. 5504 columns, K = 128 .. 50304 split 1 to 16 ways, all layouts, with
-// and without an activation, batches of 3, 6 and 12 weight gradients. What it picks among these tilings is 2.4 % behind the
-// fastest on average over 710 products (weight gradients of 1024 x 1024 over 8192 / 16384 tokens: 34.1 / 55.9 -> 29.9 /
+// and without an activation, batches of 3, 6 and 12 weight gradients. What it picks among these tilings is 1.7 % behind the
+// fastest on average over 773 products (weight gradients of 1024 x 1024 over 8192 / 16384 tokens: 34.1 / 55.9 -> 29.9 /
 // 44.2 us, of 768 x 768 over 4096: 24.7 -> 16.0); one step time for every number of tiles on a unit, and a larger tiling
 // judged at one split only, picked 6 % behind.
 double dma_us(int variant, long m, long n, long batches, int ksteps, int splits, bool a_km, bool activation, bool unaligned,
