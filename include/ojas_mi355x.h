@@ -663,6 +663,9 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * are eligible (tests and measurements). "flash_schedule": 0 = the bf16 attention kernels choose
  * between one 128-row block per workgroup and a mirrored pair by how the pairs fill the chip
  * (default), 1 / 2 = always one block / always the pair (the parity tests run both).
+ * "gemm_f32": -1 = f32 products take the tile with the least estimated time (default), 0 .. 4 = always the register-fragment
+ * kernel's 16 x 16 / 16 x 32 / 32 x 32 / 64 x 32 / 64 x 64 tile, 5 .. 8 = the direct-to-LDS kernel's 64 x 64 / 64 x 32 / 64 x 32 by
+ * two wave groups / 32 x 32 by four, wherever the operands fit it, 9 = the register-staged kernel.
  * "gemm_thin": 0 = bf16 products with at most 64 output columns over 1024 rows or
  * more go through the tiled kernels and their split-K reduce instead of the one-pass kernel for
  * thin outputs (default 1). "gemm_row_split": 0 = a product on 256x256 tiles whose last round

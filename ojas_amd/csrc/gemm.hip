@@ -457,6 +457,48 @@ int cheapest_split(int variant, long m, long n, long batches, int ksteps, int li
   return best;
 }
 
+// f32: the tile of the two kernels with the least estimated time, or neither: where direct-to-LDS loads are not possible (K no
+// whole steps, unaligned operands), large outputs are still ahead on the 128 x 128 kernel of this file, whose estimate is
+// rounds of tiles (2.4 us per 32 columns of K) and some 8 us per launch, as much again for partials and their second launch
+// when its few tiles split K. The option "gemm_f32" forces a tile that fits.
+void f32_tile(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int* frag32, int* dma32) {
+  const bool dma = omx_gemm_dma32_eligible(g, a_km, b_km);
+  const int forced = ctx->gemm_f32_tile;
+  if (forced >= FRAG32_TILES) {
+    if (forced < FRAG32_TILES + DMA32_TILES && dma) *dma32 = forced - FRAG32_TILES;
+    return;
+  }
+  double best = 1e30;
+  for (int t = 0; t < FRAG32_TILES; ++t) {
+    const double us = forced < 0 || forced == t ? omx_gemm_frag32_us(ctx, g, a_km, b_km, t) : -1.0;
+    if (us >= 0.0 && us < best) {
+      best = us;
+      *frag32 = t;
+    }
+  }
+  if (forced >= 0) return;
+  for (int t = 0; dma && t < DMA32_TILES; ++t) {
+    const double us = omx_gemm_dma32_us(ctx, g, t);
+    if (us >= 0.0 && us < best) {
+      best = us;
+      *dma32 = t;
+    }
+  }
+  if (*dma32 >= 0) *frag32 = -1;
+  if (*frag32 < 0 || dma) return;
+  // The 128 x 128 kernel with the splits that omx_gemm_impl gives it.
+  const long units = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const long tiles = static_cast<long>((g.M + 127) / 128) * ((g.N + 127) / 128) * g.batches, ksteps = (g.K + 31) / 32;
+  long splits = 1;
+  if (ksteps >= 8 && tiles < (g.batches == 1 ? 256 : 512))
+    splits = std::max(1l, std::min(((g.batches == 1 ? 512 : 1024) + tiles - 1) / tiles, ksteps / 2));
+  const long per_split = (ksteps + splits - 1) / splits;
+  splits = (ksteps + per_split - 1) / per_split;
+  const long rounds = (tiles * splits + units - 1) / units;
+  const double staged = (8.0 + (splits > 1 ? 8.0 : 0.0) + rounds * per_split * 2.4) * (b_km ? a_km ? 1.1 : 1.05 : 1.0);
+  if (staged <= best) *frag32 = -1;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
@@ -526,8 +568,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       return omx_fail(ctx, OMX_SHAPE, "%s: batch strides must be multiples of 16 bytes", op);
   }
   // Kernel choice. bf16 shapes whose output fills the chip with 256 x 256 (or
-  // 256 x 128) tiles take the direct-to-LDS kernel; everything else (f32, odd
-  // shapes, small outputs that need split-K) takes the 128 x 128 kernel.
+  // 256 x 128) tiles take the direct-to-LDS kernel; f32 shapes take f32_tile's choice;
+  // everything else (odd shapes, small outputs that need split-K) takes the 128 x 128 kernel.
   // A thin output over many rows (an adapter's rank, a gate's heads) is bound by reading A once: its
   // own kernel, which neither tiles the output nor splits K across launches.
   const bool thin = operand_dtype == OMX_BF16 && ctx->gemm_thin && !(epi && epi->mode != OMX_EPI_NONE) &&
@@ -536,10 +578,9 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   const double skinny_us = operand_dtype == OMX_BF16 && !thin && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
                                ? omx_gemm_skinny_us(ctx, g, a_km, b_km, epi && epi->mode != OMX_EPI_NONE) : -1.0;
   bool skinny = skinny_us >= 0.0;
-  // f32 outputs of less than a few rounds of 128 x 128 tiles.
-  int frag32 = -1;
+  int frag32 = -1, dma32 = -1;
   if (operand_dtype == OMX_F32 && ctx->gemm_dma_mode == 1 && !(epi && epi->mode != OMX_EPI_NONE))
-    frag32 = omx_gemm_frag32_tile(ctx, g, a_km, b_km);
+    f32_tile(ctx, g, a_km, b_km, &frag32, &dma32);
   int dma_variant = -1, small_splits = 0;
   if (!thin && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) {
     const int mode = ctx->gemm_dma_mode;
@@ -698,6 +739,10 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     const int step = dma_variant >= 9 ? 128 : 64;
     g.K = (g.k_rows + step - 1) / step * step;
   }
+  if (dma32 >= 0) {
+    omx_gemm_dma32_tile(dma32, &BM, &BN);
+    g.K = (g.k_rows + 31) / 32 * 32;
+  }
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.N + BN - 1) / BN;
   if (static_cast<long>(g.tiles_m) * g.tiles_n > 0x7fffffffl)
@@ -717,7 +762,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     // 108 tiles: two splits; of 2304 x 768, 324 tiles: two splits make three rounds of half the length).
     const long all_tiles = tiles * g.batches;
     const bool may_split =
-        !thin && !skinny && frag32 < 0 && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
+        !thin && !skinny && frag32 < 0 && dma32 < 0 && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
     if (may_split && ksteps >= 4 * min_steps && !(epi && epi->mode != OMX_EPI_NONE)) {
       splits = static_cast<int>(((g.batches == 1 ? 512 : 1024) + all_tiles - 1) / all_tiles);
       if (splits > ksteps / min_steps) splits = ksteps / min_steps;
@@ -789,6 +834,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   int32_t rc;
   if (thin) {
     rc = omx_gemm_thin_launch(ctx, g, b_km);
+  } else if (dma32 >= 0) {
+    rc = omx_gemm_dma32_launch(ctx, g, a_km, b_km, dma32);
   } else if (frag32 >= 0) {
     rc = omx_gemm_frag32_launch(ctx, g, a_km, b_km, frag32);
   } else if (skinny) {
@@ -872,6 +919,11 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value) {
     if (value != 0 && value != 1 && value != 3 && value != 4 && value != 7 && value != 8 && value != 9 && value != 10)
       return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: gemm_dma takes 0, 1, 3, 4, 7, 8, 9 or 10");
     ctx->gemm_dma_mode = static_cast<int>(value);
+    return OMX_OK;
+  }
+  if (name && strcmp(name, "gemm_f32") == 0) {
+    if (value < -1 || value > FRAG32_TILES + DMA32_TILES) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: gemm_f32 takes -1..9");
+    ctx->gemm_f32_tile = static_cast<int>(value);
     return OMX_OK;
   }
   if (name && strcmp(name, "gemm_row_split") == 0) {

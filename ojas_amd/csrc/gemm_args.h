@@ -287,6 +287,12 @@ int32_t omx_gemm_thin_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km);
 double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, bool activation);
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);
 
-// f32 kernel for small outputs: the tile it would take, or -1; the launch takes what the first returned.
-int omx_gemm_frag32_tile(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km);
+// f32 kernels: small outputs (gemm_frag32.hip) and direct-to-LDS loads (gemm_dma32.hip; g.K counts whole 32-column steps).
+// `_us`: what a tile is estimated to take; negative: not one for it.
+constexpr int FRAG32_TILES = 5, DMA32_TILES = 4;
+double omx_gemm_frag32_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
 int32_t omx_gemm_frag32_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
+bool omx_gemm_dma32_eligible(const GemmArgs& g, bool a_km, bool b_km);
+double omx_gemm_dma32_us(omx_ctx* ctx, const GemmArgs& g, int tile);
+void omx_gemm_dma32_tile(int tile, int* bm, int* bn);
+int32_t omx_gemm_dma32_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);

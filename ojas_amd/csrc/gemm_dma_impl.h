@@ -7,26 +7,6 @@
 
 namespace {
 
-// Waits until at most `groups` (up to G) groups of LPS loads are still in flight.
-template <int G, int LPS>
-__device__ __forceinline__ void wait_loads(int groups) {
-  if constexpr (G <= 0) {
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-  } else {
-    if (groups >= G) __builtin_amdgcn_s_waitcnt(vmcnt_only(G * LPS));
-    else wait_loads<G - 1, LPS>(groups);
-  }
-}
-
-// Workgroup -> tile so that the workgroups of one XCD (equal index modulo 8) take a contiguous run of the tiles, also
-// where the count is no multiple of 8: the first count % 8 XCDs have one more. 684 x 5504 over 2048 on 64 x 64 tiles,
-// 946 of them: 47.8 us in index order, where neighbours sit behind eight different L2s, 24.9 in this one; 802 products
-// of 40 .. 16384 rows 4.5 % less on average.
-__device__ inline int dma_eighth(int index, int count) {
-  const int xcd = index & 7;
-  return xcd * (count >> 3) + min(xcd, count & 7) + (index >> 3);
-}
-
 // EPI: the store pass (OMX_EPI_*). A kernel of its own per store pass keeps each one's code (a few KiB of
 // straight-line stores) and registers out of the others. TAIL: see StepBase.
 template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI, bool TAIL = false>
@@ -53,14 +33,14 @@ gemm_dma_kernel(GemmArgs g) {
   const int total = g.tiles_m * g.tiles_n;
   int split = 0, id = blockIdx.x, product = blockIdx.y;
   if (g.batches > 1 && g.splits == 1) {
-    const int r = dma_eighth(blockIdx.y * total + blockIdx.x, total * g.batches);
+    const int r = tile_of_eighth(blockIdx.y * total + blockIdx.x, total * g.batches);
     product = r / total;
     id = r - product * total;
   } else if (g.splits > 1) {
     split = blockIdx.x % g.splits;
     id = blockIdx.x / g.splits;
   } else {
-    id = dma_eighth(id, total);
+    id = tile_of_eighth(id, total);
   }
   const int band = 4;
   const int tiles_per_band = band * g.tiles_n;

@@ -4,7 +4,8 @@
 // A model a few hundred wide makes outputs of 64 Ki to a few Mi values: on 128 x 128 tiles that is 4 to 100
 // workgroups for 256 compute units, so K was split into partials and added up by a second launch, and a
 // tile's 64 matrix instructions per 32-column step ran as a chain of load, barrier, product (13 us and
-// 4 us for the second launch, whatever the size). Here a workgroup owns 16 MB x 16 NB outputs and its waves
+// 4 us for the second launch, whatever the size). gemm_dma32.hip's tiles fill the chip from some 256 x 512 outputs on; below,
+// and where a k-contiguous operand's K is not whole steps of 32, this kernel stands. Here a workgroup owns 16 MB x 16 NB outputs and its waves
 // share K, both operands go from memory straight into fragments and the waves' sums meet in LDS in wave
 // order: one launch, no partials in memory, no barrier in the loop.
 //
@@ -12,52 +13,64 @@
 // 4 g + j of the lanes' groups g = lane / 16, from both operands alike. A k-contiguous operand's lane then
 // loads 16 bytes of its row. A k-major one loads, for each j, MB (NB) adjacent rows of K row 4 g + j in one
 // piece: its blocks interleave, block m holding rows MB i + m, so one load serves every block.
-#include <algorithm>
-
 #include "gemm_tiles.h"
 
 namespace {
 
 typedef float floatx4_f __attribute__((ext_vector_type(4)));
+typedef float floatx2_f __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(1))) char* GlobalBytes;
+// A value of T at a scalar address plus the lane's offset (the empty assembly keeps the compiler from moving scalar
+// parts of the address into vector registers).
+template <typename T>
+__device__ __forceinline__ T load_at(GlobalBytes at, unsigned off) {
+  asm("" : "+s"(at));
+  return *reinterpret_cast<const __attribute__((address_space(1))) T*>(at + off);
+}
 
-// NBK blocks of 16 rows of one operand for a step: v[block][j] as above.
+// NBK blocks of 16 rows of one operand for a step: v[block][j] as above. A step's address is a scalar, the lanes add
+// 32-bit offsets that never change: with 64-bit addresses per lane and load, the multiplications of a step took a fifth
+// of the issue slots that its matrix instructions need.
 template <bool KM, int NBK>
 struct Frag32 {
-  const float* p[KM ? 1 : NBK];
-  long ld;
+  GlobalBytes base;  // the tile's first row at K = 0
+  long ld;           // bytes
+  unsigned off[KM ? 1 : NBK];
 
-  __device__ __forceinline__ void init(const float* base, long ld_, int row0, int rows, int lane) {
+  __device__ __forceinline__ void init(const float* first, long ld_, int row0, int rows, int lane) {
     const int i = lane & 15, g = lane >> 4;
-    ld = ld_;
+    ld = ld_ * 4;
+    const unsigned long long at = reinterpret_cast<unsigned long long>(first) + (KM ? row0 * 4l : row0 * ld);
+    // (tile coordinates come out of vector divisions: back to scalars)
+    const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(at));
+    const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(at >> 32));
+    base = reinterpret_cast<GlobalBytes>((static_cast<unsigned long long>(hi) << 32) | lo);
     if constexpr (KM) {
       // Whole pieces past the last row are read from it (rows is a multiple of NBK).
-      p[0] = base + min(row0 + NBK * i, rows - NBK) + static_cast<long>(4 * g) * ld;
+      off[0] = static_cast<unsigned>(min(NBK * i, rows - NBK - row0)) * 4u + static_cast<unsigned>(4 * g) * static_cast<unsigned>(ld);
     } else {
 #pragma unroll
-      for (int b = 0; b < NBK; ++b) p[b] = base + static_cast<long>(min(row0 + 16 * b + i, rows - 1)) * ld + 4 * g;
+      for (int b = 0; b < NBK; ++b)
+        off[b] = static_cast<unsigned>(min(16 * b + i, rows - 1 - row0)) * static_cast<unsigned>(ld) + 16u * g;
     }
   }
-  __device__ __forceinline__ void load(int k0, float (&v)[NBK][4]) const {
+  // Quarter `j` of a step's loads: K row 4 g + j of a k-major operand, a quarter of a k-contiguous one's blocks.
+  __device__ __forceinline__ void load(int k0, int j, float (&v)[NBK][4]) const {
     if constexpr (KM) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float* q = p[0] + static_cast<long>(k0 + j) * ld;
-        if constexpr (NBK == 4) {
-          const float4 x = *reinterpret_cast<const float4*>(q);
-          v[0][j] = x.x; v[1][j] = x.y; v[2][j] = x.z; v[3][j] = x.w;
-        } else if constexpr (NBK == 2) {
-          const float2 x = *reinterpret_cast<const float2*>(q);
-          v[0][j] = x.x; v[1][j] = x.y;
-        } else {
-          v[0][j] = *q;
-        }
+      GlobalBytes at = base + (k0 + j) * ld;
+      if constexpr (NBK == 4) {
+        const floatx4_f x = load_at<floatx4_f>(at, off[0]);
+        v[0][j] = x[0]; v[1][j] = x[1]; v[2][j] = x[2]; v[3][j] = x[3];
+      } else if constexpr (NBK == 2) {
+        const floatx2_f x = load_at<floatx2_f>(at, off[0]);
+        v[0][j] = x[0]; v[1][j] = x[1];
+      } else {
+        v[0][j] = load_at<float>(at, off[0]);
       }
-    } else {
-#pragma unroll
-      for (int b = 0; b < NBK; ++b) {
-        const float4 x = *reinterpret_cast<const float4*>(p[b] + k0);
-        v[b][0] = x.x; v[b][1] = x.y; v[b][2] = x.z; v[b][3] = x.w;
-      }
+    } else if (j * NBK % 4 == 0) {
+      const int b = j * NBK / 4;
+      const floatx4_f x = load_at<floatx4_f>(base + k0 * 4l, off[b]);
+      v[b][0] = x[0]; v[b][1] = x[1]; v[b][2] = x[2]; v[b][3] = x[3];
     }
   }
   // The last step when K is no multiple of 16: values past K are zeros and are not read.
@@ -68,8 +81,8 @@ struct Frag32 {
       const bool in = k0 + 4 * g + j < K;
 #pragma unroll
       for (int b = 0; b < NBK; ++b) {
-        if constexpr (KM) v[b][j] = in ? p[0][static_cast<long>(k0 + j) * ld + b] : 0.0f;
-        else v[b][j] = in ? p[b][k0 + j] : 0.0f;
+        if constexpr (KM) v[b][j] = in ? load_at<float>(base + (k0 + j) * ld + 4 * b, off[0]) : 0.0f;
+        else v[b][j] = in ? load_at<float>(base + (k0 + j) * 4l, off[b]) : 0.0f;
       }
     }
   }
@@ -79,9 +92,14 @@ template <bool A_KM, bool B_KM, int MB, int NB, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
   constexpr int BM = 16 * MB, BN = 16 * NB, PITCH32 = BN + 4;  // the pad keeps 16-byte pieces and spreads banks
   extern __shared__ __attribute__((aligned(16))) float sums[];  // [WAVES][BM][PITCH32]
-  gemm_select_batch(g, blockIdx.z);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
+  const int total = g.tiles_m * g.tiles_n, r = tile_of_eighth(blockIdx.x, total * g.batches);
+  const int product = r / total, id = r - product * total;
+  // An XCD's run of tiles spans the output's shorter side.
+  const int tile_m = g.tiles_m >= g.tiles_n ? id / g.tiles_n : id % g.tiles_m;
+  const int tile_n = g.tiles_m >= g.tiles_n ? id % g.tiles_n : id / g.tiles_m;
+  gemm_select_batch(g, product);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int row0 = tile_m * BM, col0 = tile_n * BN;
   Frag32<A_KM, MB> fa;
   Frag32<B_KM, NB> fb;
   fa.init(static_cast<const float*>(g.a), g.lda, row0, g.M, lane);
@@ -91,36 +109,55 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
   for (int m = 0; m < MB; ++m)
 #pragma unroll
     for (int n = 0; n < NB; ++n) acc[m][n] = floatx4_f{0.0f, 0.0f, 0.0f, 0.0f};
-  auto multiply = [&](const float (&a)[MB][4], const float (&b)[NB][4]) {
+  auto multiply = [&](const float (&a)[MB][4], const float (&b)[NB][4], int j) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int m = 0; m < MB; ++m)
-#pragma unroll
-        for (int n = 0; n < NB; ++n)
-          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[n][j], a[m][j], acc[m][n], 0, 0, 0);
+      for (int n = 0; n < NB; ++n)
+        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[n][j], a[m][j], acc[m][n], 0, 0, 0);
   };
-  constexpr int CHUNK = MB + NB <= 4 ? 4 : 2;  // steps whose loads are in flight together
+  // Sets of fragments: one in use, two on their way. A quarter of a step's loads follows each quarter of its products: all
+  // of them at once hold up the products behind them (loads between 64 and 128 products in a row: 97 and 133 us for 8192 x
+  // 256 over 2048, 84 spread; four sets: 86). 2048 x 256 over 1024: 19.4 us with the loads of two steps waited for together, 15.9.
+  constexpr int DEPTH = 3;
   const int whole = g.K / 16, steps = (g.K + 15) / 16;
   const int s_end = min(whole, steps * (wave + 1) / WAVES);
-  for (int s0 = steps * wave / WAVES; s0 < s_end; s0 += CHUNK) {
-    const int live = min(CHUNK, s_end - s0);  // uniform over the wave
-    float a[CHUNK][MB][4], b[CHUNK][NB][4];
+  int s0 = steps * wave / WAVES;
+  float a[DEPTH][MB][4], b[DEPTH][NB][4];
+  if (s0 < s_end) {
+    // No load stands behind a branch: what is in flight is known at every wait, and a step waits for its own loads only.
 #pragma unroll
-    for (int s = 0; s < CHUNK; ++s)
-      if (s < live) {
-        fa.load((s0 + s) * 16, a[s]);
-        fb.load((s0 + s) * 16, b[s]);
+    for (int d = 0; d < DEPTH - 1; ++d)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        fa.load(min(s0 + d, s_end - 1) * 16, j, a[d]);
+        fb.load(min(s0 + d, s_end - 1) * 16, j, b[d]);
       }
+#pragma unroll 1
+    for (; s0 + DEPTH <= s_end; s0 += DEPTH) {
 #pragma unroll
-    for (int s = 0; s < CHUNK; ++s)
-      if (s < live) multiply(a[s], b[s]);
+      for (int d = 0; d < DEPTH; ++d) {
+        const int to = (d + DEPTH - 1) % DEPTH, k0 = min(s0 + d + DEPTH - 1, s_end - 1) * 16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          multiply(a[d], b[d], j);
+          fa.load(k0, j, a[to]);
+          fb.load(k0, j, b[to]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+      if (s0 + d < s_end)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) multiply(a[d], b[d], j);
   }
   if (whole < steps && wave == WAVES - 1) {
-    float a[MB][4], b[NB][4];
-    fa.load_tail(whole * 16, g.K, lane, a);
-    fb.load_tail(whole * 16, g.K, lane, b);
-    multiply(a, b);
+    fa.load_tail(whole * 16, g.K, lane, a[0]);
+    fb.load_tail(whole * 16, g.K, lane, b[0]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) multiply(a[0], b[0], j);
   }
   // acc[m][n][v]: A's row i = lane % 16 of block m, B's row 4 (lane / 16) + v of block n, this wave's share of K.
   float* mine = sums + wave * (BM * PITCH32);
@@ -155,14 +192,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
 
 struct FragTile {
   int mb, nb, waves;
-  double step, fixed;  // us per 16 columns of K and per workgroup besides
+  // us: a call's first round of workgroups (fixed and per 16 columns of K), and each further round; both operands k-major.
+  double first, step, more, more_step, km_first, km_step, km_more, km_more_step;
 };
-constexpr FragTile FRAG_TILES[] = {{1, 1, 8, 0.055, 0.1}, {1, 2, 8, 0.078, 0.1}, {2, 2, 8, 0.138, 0.2}, {4, 2, 8, 0.19, 0.5}, {4, 4, 4, 0.34, 1.4}};
+constexpr FragTile FRAG_TILES[] = {{1, 1, 8, 3.10, 0.0398, 0.12, 0.0460, 2.80, 0.0529, 0.54, 0.0352},
+                                   {1, 2, 8, 3.17, 0.0613, 0.13, 0.0705, 3.16, 0.0544, 0.56, 0.0504},
+                                   {2, 2, 8, 3.21, 0.0939, 0.44, 0.1021, 3.53, 0.0800, 0.76, 0.0806},
+                                   {4, 2, 8, 3.22, 0.1761, 0.88, 0.1819, 3.55, 0.1496, 1.22, 0.1649},
+                                   {4, 4, 4, 4.71, 0.2386, 1.72, 0.3680, 4.62, 0.2546, 1.66, 0.3086}};
 
 // Whether an operand's pieces are whole and aligned for `blocks` blocks of 16 rows.
 bool frag_fits(bool km, const void* p, long ld, int rows, int blocks, long batch_bytes) {
   const long piece = km ? blocks : 4;
-  return ld % piece == 0 && (reinterpret_cast<uintptr_t>(p) & (piece * 4 - 1)) == 0 && batch_bytes % (piece * 4) == 0 &&
+  return ld % piece == 0 && ld <= 1l << 22 /* a tile's rows stay within 32 bits of bytes */ && (reinterpret_cast<uintptr_t>(p) & (piece * 4 - 1)) == 0 && batch_bytes % (piece * 4) == 0 &&
          (!km || (rows % blocks == 0 && rows >= blocks));
 }
 
@@ -173,9 +215,11 @@ int32_t launch_frag(omx_ctx* ctx, const GemmArgs& g) {
   auto kernel = &gemm_frag32_kernel<A_KM, B_KM, t.mb, t.nb, t.waves>;
   if constexpr (smem > 64 * 1024)
     OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-  dim3 grid(static_cast<unsigned>((g.N + 16 * t.nb - 1) / (16 * t.nb)), static_cast<unsigned>((g.M + 16 * t.mb - 1) / (16 * t.mb)),
-            static_cast<unsigned>(g.batches));
-  omx_launch_timed(ctx, kernel, grid, dim3(t.waves * 64), smem, ctx->timing_start, ctx->timing_stop, g);
+  GemmArgs tiled = g;
+  tiled.tiles_m = (g.M + 16 * t.mb - 1) / (16 * t.mb);
+  tiled.tiles_n = (g.N + 16 * t.nb - 1) / (16 * t.nb);
+  omx_launch_timed(ctx, kernel, dim3(static_cast<unsigned>(tiled.tiles_m) * tiled.tiles_n * g.batches), dim3(t.waves * 64), smem,
+                   ctx->timing_start, ctx->timing_stop, tiled);
   OMX_LAUNCH_CHECK(ctx, "gemm_frag32_kernel");
   return OMX_OK;
 }
@@ -192,44 +236,15 @@ int32_t launch_frag_tile(omx_ctx* ctx, const GemmArgs& g, int tile) {
 
 }  // namespace
 
-// The tile with the least estimated time, or -1 where the 128 x 128 kernel's is less still. Both estimates
-// are rounds of workgroups on the compute units times what one costs, fitted over 37 shapes from 128 x 128
-// over K = 64 to 4096 x 4096 over 1024 in three layouts: a small tile fills the chip but fetches more per
-// product (1 x 1 blocks: 0.055 us per 16 columns of K, a sixth of what 4 x 4 take for a sixteenth of the outputs);
-// the 128 x 128 tile is the cheapest per product (2.4 us per 32 columns) and pays some 8 us per launch, and as much
-// again for partials and their second launch when its few tiles split K.
-// Before and after, forward / input gradient / weight gradient layouts, us: 256 x 256 over 256: 14.3 / 14.5 / 15.6 ->
-// 3.3 each; 2048 x 256 over 256: 18.4 / 18.8 / 19.8 -> 7.2 / 6.7 / 6.6; 1024 x 256 over 2048: 30.3 / 30.7 / 31.8 ->
-// 23.3 / 21.7 / 19.1; 768 x 768 over 3072 stays (52 against 75).
-int omx_gemm_frag32_tile(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km) {
+double omx_gemm_frag32_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile) {
+  const FragTile& f = FRAG_TILES[tile];
+  if (!frag_fits(a_km, g.a, g.lda, g.M, f.mb, g.batch_a) || !frag_fits(b_km, g.b, g.ldb, g.N, f.nb, g.batch_b)) return -1.0;
   const long units = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  auto rounds = [&](long groups) { return static_cast<double>((groups + units - 1) / units); };
-  const double steps = (g.K + 15) / 16;
-  int best = -1;
-  double best_us = 1e30;
-  for (int t = 0; t < 5; ++t) {
-    const FragTile& f = FRAG_TILES[t];
-    if (!frag_fits(a_km, g.a, g.lda, g.M, f.mb, g.batch_a) || !frag_fits(b_km, g.b, g.ldb, g.N, f.nb, g.batch_b)) continue;
-    const long m = (g.M + 16 * f.mb - 1) / (16 * f.mb), n = (g.N + 16 * f.nb - 1) / (16 * f.nb);
-    if (m > 65535) continue;
-    // Two k-contiguous operands of the larger tiles fetch up to 128 pieces of 64 bytes per step.
-    const double step = t >= 3 && !a_km && !b_km ? 1.17 * f.step : f.step;
-    const double us = 2.5 + rounds(m * n * g.batches) * (steps * step + f.fixed);
-    if (us < best_us) {
-      best = t;
-      best_us = us;
-    }
-  }
-  if (best < 0) return -1;
-  // The 128 x 128 kernel with the splits that omx_gemm_impl gives it.
-  const long tiles = static_cast<long>((g.M + 127) / 128) * ((g.N + 127) / 128) * g.batches, ksteps = (g.K + 31) / 32;
-  long splits = 1;
-  if (ksteps >= 8 && tiles < (g.batches == 1 ? 256 : 512))
-    splits = std::max(1l, std::min(((g.batches == 1 ? 512 : 1024) + tiles - 1) / tiles, ksteps / 2));
-  const long per_split = (ksteps + splits - 1) / splits;
-  splits = (ksteps + per_split - 1) / per_split;
-  const double old_us = (8.0 + (splits > 1 ? 8.0 : 0.0) + rounds(tiles * splits) * per_split * 2.4) * (b_km ? a_km ? 1.1 : 1.05 : 1.0);
-  return best_us < old_us ? best : -1;
+  const long m = (g.M + 16 * f.mb - 1) / (16 * f.mb), n = (g.N + 16 * f.nb - 1) / (16 * f.nb), groups = m * n * g.batches;
+  if (groups > 0x7fffffffl) return -1.0;
+  const double more = static_cast<double>((groups + units - 1) / units - 1), steps = (g.K + 15) / 16;
+  return a_km && b_km ? f.km_first + steps * f.km_step + more * (f.km_more + steps * f.km_more_step)
+                      : f.first + steps * f.step + more * (f.more + steps * f.more_step);
 }
 
 int32_t omx_gemm_frag32_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile) {

@@ -94,6 +94,7 @@ struct omx_ctx {
   // Optional per-launch timing of the GEMM kernel (benchmark only).
   // 0: 128x128 register-staged kernel only; 1: choose by shape; others force a direct-to-LDS tiling (omx_set_option).
   int gemm_dma_mode = 1;
+  int gemm_f32_tile = -1;    // f32 products: -1: choose by estimate; 0..4, 5..8: a tile of gemm_frag32.hip, gemm_dma32.hip; 9: the register-staged kernel
   int gemm_row_split = 1;    // 0: a product whose last round of 256 x 256 tiles is mostly empty is not cut by rows
   bool gemm_in_row_split = false;  // set while omx_gemm_impl runs the two halves of a cut product
   int gemm_forced_tiling = -1;     // the tiling the first half keeps, whatever its own tile count says

@@ -583,3 +583,51 @@ def test_small_f32_outputs_share_k_between_waves(be, rows, k, n):
                                      (rows * k, k * n, rows * n))
         got = be.download(many).reshape(3, rows, n)
         assert np.abs(got - np.stack([want, -want, 2 * want])).max() <= 2 * tol
+
+
+@pytest.mark.parametrize("tile", [-1, 2, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("m,k,n", [(1, 256, 4), (64, 256, 32), (68, 288, 100), (200, 320, 516), (300, 2048, 64), (33, 256, 129), (4, 261, 8),
+                                   (132, 1000, 68), (2116, 256, 1028)])
+def test_f32_tiles(be, tile, layout, m, k, n):
+    """Every f32 tile, forced where it fits, in each operand layout: rows and columns that end inside a tile, fewer K steps
+    than stages or wave groups, reductions that end inside a step, more tiles than compute units; plain, accumulated and
+    batched outputs, against the f64 product. Rounding each of k products and k sums to f32 gives an error of at most
+    (k + 1) 2^-24 sum |a||b| per output; a value accumulated onto is one term more of the sum."""
+    from ojas_amd.backend import F32
+
+    print(f"gemm f32 tile {tile} {layout} {m}x{k}x{n}", flush=True)
+    rng = np.random.default_rng(m * 31 + k + n)
+    a, b = rng.normal(size=(2, m, k)).astype(np.float32), rng.normal(size=(2, k, n)).astype(np.float32)
+    a_km, b_km = layout[0] == "T", layout[1] == "T"
+    if (m % 4 and a_km) or (n % 4 and b_km):
+        pytest.skip("a batch's products start 16 bytes apart")
+    pad = -k % 4  # rows 16-byte aligned
+    da = be.upload(np.ascontiguousarray(a.transpose(0, 2, 1)) if a_km else np.pad(a, ((0, 0), (0, 0), (0, pad))))
+    db = be.upload(b if b_km else np.pad(np.ascontiguousarray(b.transpose(0, 2, 1)), ((0, 0), (0, 0), (0, pad))))
+    sa, sb = ((1, m) if a_km else (k + pad, 1)), ((n, 1) if b_km else (1, k + pad))
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    bound = (k + 1) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + 1e-30
+    be.set_option("gemm_f32", tile)
+    try:
+        one = be.download(be.gemm(da, sa, db, sb, m, k, n))
+        assert (np.abs(one - want[0]) <= bound[0]).all()
+        c0 = rng.normal(size=(m, n)).astype(np.float32)
+        acc = be.upload(c0)
+        be.gemm(da, sa, db, sb, m, k, n, c=acc)
+        assert (np.abs(be.download(acc) - (want[0] + c0)) <= bound[0] * (k + 2) / (k + 1) + (k + 2) * 2.0 ** -24 * np.abs(c0)).all()
+        if m * n % 4 == 0:
+            size = lambda t: int(np.prod(t.shape)) // 2
+            both = be.download(be.gemm_strided_batch(da, sa, db, sb, m, k, n, 2, (size(da), size(db), m * n))).reshape(2, m, n)
+            assert np.array_equal(both[0], one) or tile < 0
+            assert (np.abs(both - want) <= bound).all()
+        if m > 1:
+            bad = a[0].copy()
+            bad[-1, -1] = np.inf
+            dbad = be.upload(np.ascontiguousarray(bad.T) if a_km else np.pad(bad, ((0, 0), (0, pad))))
+            from ojas_amd.backend import OjasError
+            be.gemm(dbad, sa, db, sb, m, k, n)
+            with pytest.raises(OjasError):
+                be.sync()
+    finally:
+        be.set_option("gemm_f32", -1)
