@@ -48,7 +48,7 @@ GEMM_HBM_BYTES_PER_LAUNCH = {"gpt124m": 3.42e8, "gpt124m-muon": 2.75e8, "lora1b"
 # Kernel classes of omx_profile_kernels beyond the GEMM products: (bit, key, kernels, roofline).
 KERNEL_CLASSES = [
     (1, "flash_attention_forward", "flash_fwd_kernel", "mfma"),
-    (2, "flash_attention_backward", "flash_key_mean_kernel + flash_bwd_dq_kernel + flash_bwd_dkv_kernel", "mfma"),
+    (2, "flash_attention_backward", "flash_bwd_dq_kernel + flash_bwd_dkv_kernel", "mfma"),
     (3, "cross_entropy", "ce_row_fused_kernel", "hbm"),
     (4, "adamw", "adamw_apply_kernel (after adamw_check_kernel when it runs)", "hbm"),
     (5, "rms_norm_forward", "rms_fwd_vec_kernel", "hbm"),
@@ -293,7 +293,7 @@ def attention(args) -> int:
         "vs_baseline": None, "dtype": "bf16", "data": "synthetic",
         "config": {"workload": f"causal_sdpa_forward + causal_sdpa_backward: q, k, v [{b},12,1024,64] bf16",
                    "tokens_per_step": b * t},
-        "roofline": {"bound": "mfma", "kernel": "flash_fwd_kernel; flash_key_mean_kernel + flash_bwd_dq_kernel + "
+        "roofline": {"bound": "mfma", "kernel": "flash_fwd_kernel; flash_bwd_dq_kernel + "
                                                 "flash_bwd_dkv_kernel",
                      "achieved": sum(flops.values()) / total / 1e12, "peak": BF16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": sum(flops.values()) / total / 1e12 / BF16_MFMA_PEAK_TFLOPS, "traffic": None},

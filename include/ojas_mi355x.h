@@ -662,7 +662,8 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * 64x64 four-wave / 256x256 / 256x192 one-wave-per-SIMD direct-to-LDS kernel wherever the operands
  * are eligible (tests and measurements). "flash_schedule": 0 = the bf16 attention kernels choose
  * between one 128-row block per workgroup and a mirrored pair by how the pairs fill the chip
- * (default), 1 / 2 = always one block / always the pair (the parity tests run both).
+ * (default) and split a block's tiles over groups of waves where workgroups are few, 1 / 2 = always one block / always the
+ * pair, 3 / 4 = always two / four groups (two at head_dim 128; the parity tests run all).
  * "gemm_f32": -1 = f32 products take the tile with the least estimated time (default), 0 .. 4 = always the register-fragment
  * kernel's 16 x 16 / 16 x 32 / 32 x 32 / 64 x 32 / 64 x 64 tile, 5 .. 8 = the direct-to-LDS kernel's 64 x 64 / 64 x 32 / 64 x 32 by
  * two wave groups / 32 x 32 by four, wherever the operands fit it, 9 = the register-staged kernel.

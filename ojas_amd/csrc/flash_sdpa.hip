@@ -23,6 +23,7 @@
 //     keeps its k index in the matching order (bits 2 and 3 of the index
 //     swapped), so one 16-byte LDS read fetches exactly those rows.
 #include "omx_common.h"
+#include <algorithm>
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -38,6 +39,10 @@ constexpr int fpitch(int D) { return D * 2 + 16; }      // bytes per LDS row: D 
 constexpr int ftile(int D) { return 64 * fpitch(D); }   // a 64-row tile
 constexpr int FT = 256;                                 // threads per block (4 waves of 32 rows)
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr int flash_dkv_set(int D) { return 2 * ftile(D) + 2 * 64 * 4; }
+constexpr int flash_dkv_waves(int D, int groups) { return groups == 1 || (groups == 2 && D == 64) ? 2 : 1; }
+// Waves per SIMD the query-side passes are compiled for: what their LDS leaves room for.
+constexpr int flash_waves(int D, int groups) { return groups == 1 ? (D == 64 ? 3 : 2) : groups == 2 && D == 64 ? 2 : 1; }
 
 // Element strides of one tensor: between rows (time steps), heads and batches.
 struct FlashStrides {
@@ -97,52 +102,52 @@ __device__ __forceinline__ floatx16 zero16() {
   return z;
 }
 
-// A 64-row x D-column bf16 tile starting at row `row0` of a [time, D] plane: D / 32 16-byte
-// chunks per thread. Thread t moves chunk t % (D/8) of rows t / (D/8) + i * (2048 / D); rows at or
-// past `time` read as zeros.
-template <int D>
+// A 64-row x D-column bf16 tile starting at row `row0` of a [time, D] plane, moved by NT threads (a workgroup's, or a
+// key group's): 8 D / NT 16-byte chunks per thread. Thread t moves chunk t % (D/8) of rows t / (D/8) + i * (8 NT / D); rows at
+// or past `time` read as zeros.
+template <int D, int NT>
 __device__ __forceinline__ void tile_load(const unsigned short* __restrict__ plane, long rs, int row0, int time,
-                                          u32x4 (&r)[D / 32]) {
-  constexpr int CPR = D / 8, RPP = FT / CPR;
-  const int t = threadIdx.x;
+                                          u32x4 (&r)[8 * D / NT]) {
+  constexpr int CPR = D / 8, RPP = NT / CPR;
+  const int t = threadIdx.x % NT;
   const int row = row0 + t / CPR, kc = t % CPR;
 #pragma unroll
-  for (int i = 0; i < D / 32; ++i) {
+  for (int i = 0; i < 8 * D / NT; ++i) {
     r[i] = u32x4{0u, 0u, 0u, 0u};
     if (row + i * RPP < time)
       r[i] = *reinterpret_cast<const u32x4*>(plane + static_cast<long>(row + i * RPP) * rs + kc * 8);
   }
 }
 // [row][d] form.
-template <int D>
-__device__ __forceinline__ void tile_store_rows(char* lds, const u32x4 (&r)[D / 32]) {
-  constexpr int CPR = D / 8, RPP = FT / CPR;
-  const int t = threadIdx.x;
+template <int D, int NT>
+__device__ __forceinline__ void tile_store_rows(char* lds, const u32x4 (&r)[8 * D / NT]) {
+  constexpr int CPR = D / 8, RPP = NT / CPR;
+  const int t = threadIdx.x % NT;
   const int row = t / CPR, kc = t % CPR;
 #pragma unroll
-  for (int i = 0; i < D / 32; ++i) *reinterpret_cast<u32x4*>(lds + (row + i * RPP) * fpitch(D) + kc * 16) = r[i];
+  for (int i = 0; i < 8 * D / NT; ++i) *reinterpret_cast<u32x4*>(lds + (row + i * RPP) * fpitch(D) + kc * 16) = r[i];
 }
 // The same loads with the per-thread part of the address formed once. A tile that ends inside the
 // sequence is fetched from a wave-uniform base (plane + row0 rows) plus the thread's fixed 32-bit byte
 // offset: no address arithmetic and no bounds test per load. Only the last, ragged tile takes the
 // checked path. The host refuses row strides for which the offset would not fit.
-template <int D>
+template <int D, int NT>
 struct TileFetch {
-  static constexpr int CPR = D / 8, RPP = FT / CPR;
+  static constexpr int CPR = D / 8, RPP = NT / CPR;
   unsigned off;  // bytes from a tile's first element to this thread's first chunk
   long rs;
   int time;
   __device__ __forceinline__ TileFetch(long row_stride, int t_end) : rs(row_stride), time(t_end) {
-    const int t = threadIdx.x;
+    const int t = threadIdx.x % NT;
     off = static_cast<unsigned>((t / CPR) * row_stride + (t % CPR) * 8) * 2u;
   }
-  __device__ __forceinline__ void load(const unsigned short* __restrict__ plane, int row0, u32x4 (&r)[D / 32]) const {
+  __device__ __forceinline__ void load(const unsigned short* __restrict__ plane, int row0, u32x4 (&r)[8 * D / NT]) const {
     if (row0 + 64 <= time) {
       const char* base = reinterpret_cast<const char*>(plane + static_cast<long>(row0) * rs);
 #pragma unroll
-      for (int i = 0; i < D / 32; ++i) r[i] = *reinterpret_cast<const u32x4*>(base + static_cast<long>(i * RPP) * rs * 2 + off);
+      for (int i = 0; i < 8 * D / NT; ++i) r[i] = *reinterpret_cast<const u32x4*>(base + static_cast<long>(i * RPP) * rs * 2 + off);
     } else {
-      tile_load<D>(plane, rs, row0, time, r);
+      tile_load<D, NT>(plane, rs, row0, time, r);
     }
   }
 };
@@ -383,23 +388,28 @@ __device__ __forceinline__ void flash_fwd_tile(const char* k_rows, const char* v
 
 // WIN: the sliding-window form (every tile tested element by element), compiled apart so that the
 // plain causal kernel carries neither its code nor its registers.
-template <int D, typename TO, bool WIN>
-__global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_fwd_kernel(const unsigned short* __restrict__ q,
+// GROUPS > 1: the workgroup's waves form that many groups, which take the key tiles of 128 / GROUPS query rows in turn and
+// meet in LDS at the end (flash_groups says when).
+template <int D, typename TO, bool WIN, int GROUPS>
+__global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_fwd_kernel(const unsigned short* __restrict__ q,
                                                        const unsigned short* __restrict__ k,
                                                        const unsigned short* __restrict__ v, TO* __restrict__ out,
                                                        unsigned short* __restrict__ resid, float* __restrict__ lse,
                                                        FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
-  constexpr int KK = D / 16, MT = D / 32, NL = D / 32;  // d slabs, d blocks of the output, loads per thread and tile
-  // Two key / value tile pairs: the next tile is stored while this one is multiplied, so a tile
+  constexpr int NT = FT / GROUPS, ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;  // threads and waves of a group, rows of a block
+  constexpr int KK = D / 16, MT = D / 32, NL = 8 * D / NT;  // d slabs, d blocks of the output, loads per thread and tile
+  // Two key / value tile pairs (per group): the next tile is stored while this one is multiplied, so a tile
   // costs one barrier.
-  __shared__ __attribute__((aligned(16))) char smem[4 * ftile(D)];
-  const int lane = threadIdx.x & 63, wave = wave_index(), l32 = lane & 31, lg = lane >> 5;
+  __shared__ __attribute__((aligned(16))) char flash_lds[GROUPS * 4 * ftile(D)];
+  const int lane = threadIdx.x & 63, l32 = lane & 31, lg = lane >> 5;
+  const int group = GROUPS == 1 ? 0 : wave_index() / ROW_WAVES, wave = GROUPS == 1 ? wave_index() : wave_index() % ROW_WAVES;
+  char* const smem = flash_lds + group * (4 * ftile(D));
   const int T = s.time;
-  const TileFetch<D> fetch(s.kv.rs, T);
+  const TileFetch<D, NT> fetch(s.kv.rs, T);
   // Query block j sees j / 2 + 1 key tiles (causal): a workgroup takes a late block and then
   // its mirror image from the front, so every workgroup does the same amount of work and the
   // grid ends without a tail of half-empty compute units.
-  const int q_blocks = (T + 127) / 128;
+  const int q_blocks = (T + ROWS - 1) / ROWS;
   int pair;
   long plane;
   if (s.q_single) {  // block rank (0 = the last, heaviest block) in the high part of the index
@@ -416,7 +426,7 @@ __global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_fwd_kernel(const un
     const unsigned short* qp = q + b * s.q.bs + h * s.q.hs;
     const unsigned short* kp = k + b * s.kv.bs + kvh * s.kv.hs;
     const unsigned short* vp = v + b * s.kv.bs + kvh * s.kv.hs;
-    const int wave_q0 = qb * 128 + wave * 32;
+    const int wave_q0 = qb * ROWS + wave * 32;
     const int q_row = wave_q0 + l32;
     u32x4 qf[KK];
     row_frags<D>(qp, s.q.rs, q_row, T, lg, qf);
@@ -431,45 +441,48 @@ __global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_fwd_kernel(const un
     // come through scaled by (sum of rounded weights) / (sum of weights).
     float m = -INFINITY, lsum = 0.0f, wsum = 0.0f;
     const float scale_log2 = s.scale * LOG2E;
-    const int block_q0 = qb * 128, block_q1 = min(T - 1, qb * 128 + 127);
+    const int block_q0 = qb * ROWS, block_q1 = min(T - 1, qb * ROWS + ROWS - 1);
     const int kt_first = s.window > 0 ? max(0, block_q0 + 1 - s.window) / 64 : 0;
     const int kt_last = block_q1 / 64;
+    // The tiles of this group: kt0, kt0 + GROUPS, ... (a group without one reads the first tile and leaves it).
+    const int kt0 = kt_first + group;
     // The next tile's global loads are in flight while the current one is multiplied.
     u32x4 rk[NL], rv[NL];
-    fetch.load(kp, kt_first * 64, rk);
-    fetch.load(vp, kt_first * 64, rv);
+    fetch.load(kp, min(kt0, kt_last) * 64, rk);
+    fetch.load(vp, min(kt0, kt_last) * 64, rv);
     __syncthreads();  // the previous pass's reads of the first pair are done
-    tile_store_rows<D>(smem, rk);
-    tile_store_rows<D>(smem + ftile(D), rv);
-    if (kt_first < kt_last) {
-      fetch.load(kp, kt_first * 64 + 64, rk);
-      fetch.load(vp, kt_first * 64 + 64, rv);
+    tile_store_rows<D, NT>(smem, rk);
+    tile_store_rows<D, NT>(smem + ftile(D), rv);
+    if (kt0 + GROUPS <= kt_last) {
+      fetch.load(kp, (kt0 + GROUPS) * 64, rk);
+      fetch.load(vp, (kt0 + GROUPS) * 64, rv);
     }
     // One step of the tile pipeline, taken by every wave for every tile of the block: wait for tile
     // kt's pair, store tile kt + 1 into the other pair, start the loads of tile kt + 2.
     const char* k_rows;
     const char* v_rows;
     auto advance = [&](int kt) {
-      const int cur = (kt - kt_first) & 1;
+      const int cur = GROUPS == 1 ? (kt - kt_first) & 1 : (kt - kt0) / GROUPS & 1;
       k_rows = smem + cur * 2 * ftile(D);
       v_rows = k_rows + ftile(D);
       __syncthreads();  // this pair is complete, and every wave is done with the other one
-      if (kt < kt_last) {
+      if (kt + GROUPS <= kt_last) {
         char* next = smem + (cur ^ 1) * 2 * ftile(D);
-        tile_store_rows<D>(next, rk);
-        tile_store_rows<D>(next + ftile(D), rv);
-        if (kt + 1 < kt_last) {
-          fetch.load(kp, kt * 64 + 128, rk);
-          fetch.load(vp, kt * 64 + 128, rv);
+        tile_store_rows<D, NT>(next, rk);
+        tile_store_rows<D, NT>(next + ftile(D), rv);
+        if (kt + 2 * GROUPS <= kt_last) {
+          fetch.load(kp, (kt + 2 * GROUPS) * 64, rk);
+          fetch.load(vp, (kt + 2 * GROUPS) * 64, rv);
         }
       }
     };
-    int kt = kt_first;
+    int kt = kt0;
+    const int kt_end = kt_last + group;  // every group takes as many steps as the first
     if constexpr (WIN) {
-      for (; kt <= kt_last; ++kt) {
+      for (; kt <= kt_end; kt += GROUPS) {
         advance(kt);
         const int key0 = kt * 64;
-        if (key0 <= wave_q0 + 31 && key0 + 63 + s.window > wave_q0)
+        if ((GROUPS == 1 || kt <= kt_last) && key0 <= wave_q0 + 31 && key0 + 63 + s.window > wave_q0)
           flash_fwd_tile<D, 2, -1, true>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, s.window, lane);
       }
     } else if (wave_q0 < T) {  // (a wave whose rows all lie past the sequence end only keeps the barriers)
@@ -479,21 +492,67 @@ __global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_fwd_kernel(const un
       // the tile that starts 32 keys earlier. The tiles before it need no mask, and their loop holds
       // nothing else: one body, so the accumulators stay in the registers the matrix units update.
       const int diag_kt = wave_q0 / 64;
-      for (; kt < diag_kt; ++kt) {
+      for (; kt < diag_kt; kt += GROUPS) {
         advance(kt);
         flash_fwd_tile<D, 2, -1, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, kt * 64, q_row, T, 0, lane);
       }
-      advance(kt);
-      const int key0 = kt * 64;
-      if (D > 64 || key0 + 63 >= T)  // (at head_dim 128 the two cut-tile forms cost registers the kernel does not have)
-        flash_fwd_tile<D, 2, -1, true>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
-      else if (key0 == wave_q0)
-        flash_fwd_tile<D, 1, 0, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
-      else
-        flash_fwd_tile<D, 2, 1, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
-      ++kt;
+      if (GROUPS == 1 || kt == diag_kt) {
+        advance(kt);
+        const int key0 = kt * 64;
+        if (D > 64 || key0 + 63 >= T)  // (at head_dim 128 the two cut-tile forms cost registers the kernel does not have)
+          flash_fwd_tile<D, 2, -1, true>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
+        else if (key0 == wave_q0)
+          flash_fwd_tile<D, 1, 0, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
+        else
+          flash_fwd_tile<D, 2, 1, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
+        kt += GROUPS;
+      }
     }
-    for (; kt <= kt_last; ++kt) advance(kt);  // tiles of the block's later waves (same barrier count for all)
+    for (; kt <= kt_end; kt += GROUPS) advance(kt);  // tiles of the block's later waves (same barrier count for all)
+    if constexpr (GROUPS > 1) {
+      // The groups' weights and sums, moved to one reference point per row.
+      constexpr int PART = (MT * 16 + 3) * 64;  // floats of a wave
+      float* const meet = reinterpret_cast<float*>(flash_lds);
+      __syncthreads();  // every wave is done with the tiles
+      if (group > 0) {
+        float* mine = meet + ((group - 1) * ROW_WAVES + wave) * PART + lane;
+        mine[0] = m;
+        mine[64] = lsum;
+        mine[128] = wsum;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int vv = 0; vv < 16; ++vv) mine[(3 + mt * 16 + vv) * 64] = o[mt][vv];
+      }
+      __syncthreads();
+      if (group > 0) return;
+      const float* parts[GROUPS - 1];
+      float top = m;
+#pragma unroll
+      for (int g = 0; g < GROUPS - 1; ++g) {
+        parts[g] = meet + (g * ROW_WAVES + wave) * PART + lane;
+        top = fmaxf(top, parts[g][0]);
+      }
+      const float neg_top = top == -INFINITY ? 0.0f : -top * scale_log2;
+      const float own = __builtin_amdgcn_exp2f(fmaf(m, scale_log2, neg_top));
+      lsum *= own;
+      wsum *= own;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int vv = 0; vv < 16; ++vv) o[mt][vv] *= own;
+#pragma unroll
+      for (int g = 0; g < GROUPS - 1; ++g) {
+        const float w = __builtin_amdgcn_exp2f(fmaf(parts[g][0], scale_log2, neg_top));
+        lsum = fmaf(parts[g][64], w, lsum);
+        wsum = fmaf(parts[g][128], w, wsum);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int vv = 0; vv < 16; ++vv) o[mt][vv] = fmaf(parts[g][(3 + mt * 16 + vv) * 64], w, o[mt][vv]);
+      }
+      m = top;
+    }
     wsum = halves_sum(wsum);
     bool bad = false;
     if (q_row < T) {
@@ -514,13 +573,13 @@ __global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_fwd_kernel(const un
 // ------------------------------------------------------------------ backward: dK, dV
 // One 64-query x 32-key tile of one wave in the dK/dV pass. GENERAL: the tile crosses the diagonal,
 // the sequence end or a window edge and every element is tested (as in the dQ pass, the cheaper
-// forms of the cut tile would push the kernel past its registers).
-template <int D, bool WANT_DK, bool WANT_DV, bool GENERAL>
+// forms of the cut tile would push the kernel past its registers): 0 / 1: no / yes, 2: as `cut` says.
+template <int D, bool WANT_DK, bool WANT_DV, int GENERAL>
 __device__ __forceinline__ void flash_dkv_tile(const char* q_rows, const char* g_rows, const float* lse_s,
                                                const float* del_s, const u32x4 (&kf)[D / 16],
                                                const u32x4 (&vf)[WANT_DK ? D / 16 : 1], floatx16 (&dk)[WANT_DK ? D / 32 : 1],
                                                floatx16 (&dv)[WANT_DV ? D / 32 : 1], float scale_log2, int q0, int key_row,
-                                               int T, int window, int lane) {
+                                               int T, int window, int lane, bool cut = true) {
   constexpr int KK = D / 16, MT = D / 32;
   const int l32 = lane & 31, lg = lane >> 5;
 #pragma unroll
@@ -531,7 +590,7 @@ __device__ __forceinline__ void flash_dkv_tile(const char* q_rows, const char* g
       sc = mfma(frag_rows<D>(q_rows, sub, kk, l32, lg), kf[kk], sc);
       if constexpr (WANT_DK) dp = mfma(frag_rows<D>(g_rows, sub, kk, l32, lg), vf[kk], dp);
     }
-    if constexpr (GENERAL) {
+    if (GENERAL == 1 || (GENERAL == 2 && cut)) {
 #pragma unroll
       for (int vv = 0; vv < 16; ++vv) {
         const int qi = q0 + sub * 32 + acc_row(vv, lg);
@@ -579,20 +638,24 @@ __device__ __forceinline__ void flash_dkv_tile(const char* q_rows, const char* g
 // once for both. At head_dim 128 the two accumulator sets (128 registers), both key / value
 // fragments (64) and the score tiles do not fit the 256 registers of two waves per SIMD, so the
 // block is walked twice, once per gradient; the second walk recomputes the scores.
-template <int D, typename TO, bool WANT_DK, bool WANT_DV, bool WIN>
+// GROUPS > 1: groups of the waves take the query tiles of 128 / GROUPS keys in turn, as in the forward.
+template <int D, typename TO, bool WANT_DK, bool WANT_DV, bool WIN, int GROUPS>
 __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict__ q,
                                                 const unsigned short* __restrict__ k,
                                                 const unsigned short* __restrict__ v, const float* __restrict__ lse,
                                                 const float* __restrict__ delta, const unsigned short* __restrict__ gy,
-                                                TO* __restrict__ gk, TO* __restrict__ gv, const FlashShape& s, char* smem,
+                                                TO* __restrict__ gk, TO* __restrict__ gv, const FlashShape& s, char* lds,
                                                 int kb, int b, int gidx) {
-  constexpr int KK = D / 16, MT = D / 32, NL = D / 32;
-  constexpr int SET = 2 * ftile(D) + 2 * 64 * 4;
-  const int lane = threadIdx.x & 63, wave = wave_index(), l32 = lane & 31, lg = lane >> 5;
+  constexpr int NT = FT / GROUPS, ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;
+  constexpr int KK = D / 16, MT = D / 32, NL = 8 * D / NT;
+  constexpr int SET = flash_dkv_set(D);
+  const int lane = threadIdx.x & 63, l32 = lane & 31, lg = lane >> 5, tid = threadIdx.x % NT;
+  const int group = GROUPS == 1 ? 0 : wave_index() / ROW_WAVES, wave = GROUPS == 1 ? wave_index() : wave_index() % ROW_WAVES;
+  char* const smem = lds + group * (2 * SET);
   const int T = s.time;
-  const TileFetch<D> fetch_q(s.q.rs, T), fetch_g(s.o.rs, T);
+  const TileFetch<D, NT> fetch_q(s.q.rs, T), fetch_g(s.o.rs, T);
   const long kv_off = b * s.kv.bs + gidx * s.kv.hs;
-  const int wave_k0 = kb * 128 + wave * 32;
+  const int wave_k0 = kb * ROWS + wave * 32;
   const int key_row = wave_k0 + l32;
   u32x4 kf[KK], vf[WANT_DK ? KK : 1];
   row_frags<D>(k + kv_off, s.kv.rs, key_row, T, lg, kf);
@@ -603,43 +666,51 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
 #pragma unroll
   for (int mt = 0; mt < (WANT_DV ? MT : 1); ++mt) dv[mt] = zero16();
   const float scale_log2 = s.scale * LOG2E;
-  const int block_k0 = kb * 128, block_k1 = min(T - 1, kb * 128 + 127);
+  const int block_k0 = kb * ROWS, block_k1 = min(T - 1, kb * ROWS + ROWS - 1);
   const int qt_first = block_k0 / 64;
   const int qt_last = (s.window > 0 ? min(T - 1, block_k1 + s.window - 1) : T - 1) / 64;
   bool bad = false;
   // One flat sequence of (query head of the group, query tile), ascending, so the
   // next tile's global loads can be in flight while the current one is multiplied.
   const int nq = qt_last - qt_first + 1;
-  const int steps = s.rep * nq;
+  const int steps = (s.rep * nq - group + GROUPS - 1) / GROUPS;  // this group's: GROUPS tiles apart
   u32x4 rq[NL], rg[NL];
   float row_lse = 0.0f, row_del = 0.0f;
   // (head of the group, query tile) of the tile being fetched.
   int fetch_r = 0, fetch_qt = qt_first;
+  auto skip = [&](int& r, int& qt, int tiles) {
+#pragma unroll
+    for (int i = 0; i < tiles; ++i)
+      if (++qt > qt_last) {
+        qt = qt_first;
+        ++r;
+      }
+  };
+  if constexpr (GROUPS > 1) {
+    for (int i = 0; i < group; ++i) skip(fetch_r, fetch_qt, 1);
+  }
   auto fetch = [&]() {
-    const int r = fetch_r, q0 = fetch_qt * 64;
-    if (++fetch_qt > qt_last) {
-      fetch_qt = qt_first;
-      ++fetch_r;
-    }
+    const int r = GROUPS == 1 ? fetch_r : min(fetch_r, s.rep - 1), q0 = fetch_qt * 64;
+    skip(fetch_r, fetch_qt, GROUPS);
     const long q_plane = static_cast<long>(b) * s.heads + static_cast<long>(gidx) * s.rep + r;
     const long head = static_cast<long>(gidx) * s.rep + r;
     fetch_q.load(q + b * s.q.bs + head * s.q.hs, q0, rq);
     fetch_g.load(gy + b * s.o.bs + head * s.o.hs, q0, rg);
     row_lse = 0.0f;
     row_del = 0.0f;
-    if (threadIdx.x < 64 && q0 + static_cast<int>(threadIdx.x) < T) {
-      row_lse = lse[q_plane * T + q0 + threadIdx.x];
-      row_del = delta[q_plane * T + q0 + threadIdx.x];
+    if (tid < 64 && q0 + tid < T) {
+      row_lse = lse[q_plane * T + q0 + tid];
+      row_del = delta[q_plane * T + q0 + tid];
       bad |= !(dev_finite(row_lse) && dev_finite(row_del));
     }
   };
   auto store_set = [&](char* set) {
-    tile_store_rows<D>(set, rq);
-    tile_store_rows<D>(set + ftile(D), rg);
-    if (threadIdx.x < 64) {
+    tile_store_rows<D, NT>(set, rq);
+    tile_store_rows<D, NT>(set + ftile(D), rg);
+    if (tid < 64) {
       float* stats = reinterpret_cast<float*>(set + 2 * ftile(D));
-      stats[threadIdx.x] = row_lse * LOG2E;
-      stats[64 + threadIdx.x] = row_del;
+      stats[tid] = row_lse * LOG2E;
+      stats[64 + tid] = row_del;
     }
   };
   fetch();
@@ -665,11 +736,51 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     }
     ++idx;
   };
-  auto tile = [&](auto general, int q0) {
+  auto tile = [&](auto general, int q0, bool cut = true) {
     flash_dkv_tile<D, WANT_DK, WANT_DV, decltype(general)::value>(q_rows, g_rows, lse_s, del_s, kf, vf, dk, dv, scale_log2, q0,
-                                                                 key_row, T, s.window, lane);
+                                                                 key_row, T, s.window, lane, cut);
   };
-  for (int r = 0; r < s.rep; ++r) {
+  if constexpr (GROUPS > 1) {
+    int r = 0, qt = qt_first;
+    for (int i = 0; i < group; ++i) skip(r, qt, 1);
+    const int rounds = (s.rep * nq + GROUPS - 1) / GROUPS;
+    for (int i = 0; i < rounds; ++i) {
+      advance();
+      const int q0 = qt * 64;
+      if (r < s.rep && wave_k0 < T && q0 + 63 >= wave_k0 && (!WIN || q0 < wave_k0 + 31 + s.window)) {
+        if constexpr (WIN) tile(std::true_type{}, q0);
+        else tile(std::integral_constant<int, 2>{}, q0, q0 < wave_k0 + 32 || q0 + 64 > T || wave_k0 + 31 >= T);
+      }
+      skip(r, qt, GROUPS);
+    }
+    constexpr int PART = ((WANT_DK ? MT : 0) + (WANT_DV ? MT : 0)) * 16 * 64;  // floats of a wave
+    float* const meet = reinterpret_cast<float*>(lds);
+    __syncthreads();  // every wave is done with the tiles
+    if (group > 0) {
+      float* mine = meet + ((group - 1) * ROW_WAVES + wave) * PART + lane;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int vv = 0; vv < 16; ++vv) {
+          if constexpr (WANT_DK) mine[(mt * 16 + vv) * 64] = dk[mt][vv];
+          if constexpr (WANT_DV) mine[((WANT_DK ? MT : 0) * 16 + mt * 16 + vv) * 64] = dv[mt][vv];
+        }
+    }
+    __syncthreads();
+    if (group > 0) return bad;
+#pragma unroll
+    for (int g = 0; g < GROUPS - 1; ++g) {
+      const float* part = meet + (g * ROW_WAVES + wave) * PART + lane;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int vv = 0; vv < 16; ++vv) {
+          if constexpr (WANT_DK) dk[mt][vv] += part[(mt * 16 + vv) * 64];
+          if constexpr (WANT_DV) dv[mt][vv] += part[((WANT_DK ? MT : 0) * 16 + mt * 16 + vv) * 64];
+        }
+    }
+  }
+  for (int r = 0; GROUPS == 1 && r < s.rep; ++r) {
     int qt = qt_first;
     if constexpr (WIN) {
       for (; qt <= qt_last; ++qt) {
@@ -703,17 +814,17 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
   return bad;
 }
 
-template <int D, typename TO, bool WIN>
-__global__ __launch_bounds__(FT, 2) void flash_bwd_dkv_kernel(
+template <int D, typename TO, bool WIN, int GROUPS>
+__global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_dkv_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const float* __restrict__ lse, const float* __restrict__ delta, const unsigned short* __restrict__ gy,
     TO* __restrict__ gk, TO* __restrict__ gv, FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
   // Two sets of (query tile, gradient tile, 64 log-sum-exp values, 64 row terms): the next set is
   // stored while this one is multiplied, so a tile costs one barrier.
-  __shared__ __attribute__((aligned(16))) char smem[2 * (2 * ftile(D) + 2 * 64 * 4)];
+  __shared__ __attribute__((aligned(16))) char smem[GROUPS * 2 * flash_dkv_set(D)];
   // Early key blocks are seen by the most queries: a workgroup takes one of them and then its
   // mirror image from the back (see the forward kernel).
-  const int k_blocks = (s.time + 127) / 128;
+  const int k_blocks = (s.time + 128 / GROUPS - 1) / (128 / GROUPS);
   int pair;
   long kv_plane;
   if (s.kv_single) {  // block index (0 = the first, heaviest block) in the high part of the index
@@ -728,51 +839,46 @@ __global__ __launch_bounds__(FT, 2) void flash_bwd_dkv_kernel(
     const int kb = pass == 0 ? pair : k_blocks - 1 - pair;
     if (pass == 1 && kb <= pair) break;
     if constexpr (D == 64) {
-      bad |= flash_dkv_block<D, TO, true, true, WIN>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
+      bad |= flash_dkv_block<D, TO, true, true, WIN, GROUPS>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
     } else {
-      bad |= flash_dkv_block<D, TO, false, true, WIN>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
-      bad |= flash_dkv_block<D, TO, true, false, WIN>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
+      bad |= flash_dkv_block<D, TO, false, true, WIN, GROUPS>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
+      bad |= flash_dkv_block<D, TO, true, false, WIN, GROUPS>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
     }
   }
   if (bad) dev_raise_fault(fault, tag);
 }
 
-// ------------------------------------------------------------------ backward: the mean key row
-// key_mean[b, kv head, :] = the mean of up to 64 of that head's key rows, evenly spaced in time, in
-// f32. The dQ pass needs a vector close to what the key rows share, not the exact mean (what it
-// does with it is exact for any vector), so a sample is enough. One workgroup per (batch, kv head);
-// a lane reads 8 values of a row, 256 / (D / 8) rows go round at once.
+// ------------------------------------------------------------------ backward: dQ
+// This thread's share of the sum of up to 64 of a head's key rows, evenly spaced in time: part[row group][D]. The dQ pass
+// needs a vector close to what the key rows share, not their exact mean (what it does with it is exact for any vector), so
+// a sample is enough; every workgroup takes its own (8 KiB out of L2 beside its tiles; a launch of its own before the
+// pass cost 2 to 5 us). A thread reads 8 values of a row, 256 / (D / 8) rows go round at once.
 template <int D>
-__global__ __launch_bounds__(256) void flash_key_mean_kernel(const unsigned short* __restrict__ k,
-                                                             float* __restrict__ key_mean, FlashShape s) {
-  constexpr int LPR = D / 8, ROWS = 256 / LPR;
-  __shared__ float part[ROWS][D];
-  const int b = blockIdx.x / s.kv_heads, h = blockIdx.x % s.kv_heads;
-  const unsigned short* kp = k + b * s.kv.bs + h * s.kv.hs;
-  const int col = (threadIdx.x % LPR) * 8, first = threadIdx.x / LPR;
-  const int samples = min(s.time, 64);
+__device__ __forceinline__ void key_sample_sum(const unsigned short* __restrict__ kp, long rs, int time, float* part) {
+  constexpr int LPR = D / 8, ROWS = FT / LPR;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (the sample's addresses, formed ahead of the blocks' loop, would cost the loop registers)
+  const int col = (tid % LPR) * 8, first = tid / LPR;
+  const int samples = min(time, 64);
   float sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int i = first; i < samples; i += ROWS) {
-    const long row = static_cast<long>(i) * s.time / samples;
-    const u32x4 w = *reinterpret_cast<const u32x4*>(kp + row * s.kv.rs + col);
-    const unsigned int ww[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      sum[2 * j] += __uint_as_float(ww[j] << 16);
-      sum[2 * j + 1] += __uint_as_float(ww[j] & 0xffff0000u);
+  for (int n = 0; n < 64 / ROWS; ++n) {
+    const int i = first + n * ROWS;
+    if (i < samples) {
+      const long row = static_cast<long>(i) * time / samples;
+      const u32x4 w = *reinterpret_cast<const u32x4*>(kp + row * rs + col);
+      const unsigned int ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        sum[2 * j] += __uint_as_float(ww[j] << 16);
+        sum[2 * j + 1] += __uint_as_float(ww[j] & 0xffff0000u);
+      }
     }
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) part[first][col + i] = sum[i];
-  __syncthreads();
-  if (threadIdx.x < D) {
-    float total = 0.0f;
-    for (int r = 0; r < ROWS; ++r) total += part[r][threadIdx.x];
-    key_mean[static_cast<long>(blockIdx.x) * D + threadIdx.x] = total / static_cast<float>(samples);
-  }
+  for (int i = 0; i < 8; ++i) part[first * D + col + i] = sum[i];
 }
 
-// ------------------------------------------------------------------ backward: dQ
 // One 32-query x 64-key tile of one wave in the dQ pass. GENERAL: the tile crosses the diagonal,
 // the sequence end or a window edge and every element is tested (the forward's cheaper forms of
 // the cut tile cost registers this kernel does not have: with them it spills, and runs 11 % slower).
@@ -816,20 +922,23 @@ __device__ __forceinline__ void flash_dq_tile(const char* k_rows, const char* v_
   }
 }
 
-template <int D, typename TO, bool WIN>
-__global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_bwd_dq_kernel(
+template <int D, typename TO, bool WIN, int GROUPS>
+__global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_bwd_dq_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const unsigned short* __restrict__ out, const unsigned short* __restrict__ resid, const float* __restrict__ lse,
-    float* __restrict__ delta, const float* __restrict__ key_mean, const unsigned short* __restrict__ gy,
-    TO* __restrict__ gq, FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
-  constexpr int KK = D / 16, MT = D / 32, NL = D / 32;
-  // Two key / value tile pairs, as in the forward: one barrier per tile.
-  __shared__ __attribute__((aligned(16))) char smem[4 * ftile(D)];
-  const int lane = threadIdx.x & 63, wave = wave_index(), l32 = lane & 31, lg = lane >> 5;
+    float* __restrict__ delta, const unsigned short* __restrict__ gy, TO* __restrict__ gq, FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
+  constexpr int NT = FT / GROUPS, ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;
+  constexpr int KK = D / 16, MT = D / 32, NL = 8 * D / NT;
+  // Two key / value tile pairs (per group), as in the forward: one barrier per tile.
+  __shared__ __attribute__((aligned(16))) char flash_lds[GROUPS * 4 * ftile(D)];
+  __shared__ __attribute__((aligned(16))) float mean_key[D];
+  const int lane = threadIdx.x & 63, l32 = lane & 31, lg = lane >> 5;
+  const int group = GROUPS == 1 ? 0 : wave_index() / ROW_WAVES, wave = GROUPS == 1 ? wave_index() : wave_index() % ROW_WAVES;
+  char* const smem = flash_lds + group * (4 * ftile(D));
   const int T = s.time;
-  const TileFetch<D> fetch(s.kv.rs, T);
+  const TileFetch<D, NT> fetch(s.kv.rs, T);
   // A late query block, then its mirror image from the front (see the forward kernel).
-  const int q_blocks = (T + 127) / 128;
+  const int q_blocks = (T + ROWS - 1) / ROWS;
   int pair;
   long plane;
   if (s.q_single) {  // block rank (0 = the last, heaviest block) in the high part of the index
@@ -845,7 +954,7 @@ __global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_bwd_dq_kernel(
     const int kvh = h / s.rep;
     const unsigned short* kp = k + b * s.kv.bs + kvh * s.kv.hs;
     const unsigned short* vp = v + b * s.kv.bs + kvh * s.kv.hs;
-    const int wave_q0 = qb * 128 + wave * 32;
+    const int wave_q0 = qb * ROWS + wave * 32;
     const int q_row = wave_q0 + l32;
     u32x4 qf[KK], gf[KK];
     row_frags<D>(q + b * s.q.bs + h * s.q.hs, s.q.rs, q_row, T, lg, qf);
@@ -879,7 +988,7 @@ __global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_bwd_dq_kernel(
     bool bad = false;
     if (q_row < T) {
       row_lse = lse[plane * T + q_row];
-      if (lg == 0) delta[plane * T + q_row] = row_del;
+      if (lg == 0 && group == 0) delta[plane * T + q_row] = row_del;
       bad |= !(dev_finite(row_lse) && dev_finite(row_del));
     }
     const float neg_lse = -row_lse * LOG2E;
@@ -893,66 +1002,104 @@ __global__ __launch_bounds__(FT, D == 64 ? 3 : 2) void flash_bwd_dq_kernel(
     // lane's share of the row sum of the rounded dS; the end takes (row sum) x (mean key) off.
     float ds_sum = 0.0f;
     const float scale_log2 = s.scale * LOG2E;
-    const int block_q0 = qb * 128, block_q1 = min(T - 1, qb * 128 + 127);
+    const int block_q0 = qb * ROWS, block_q1 = min(T - 1, qb * ROWS + ROWS - 1);
     const int kt_first = s.window > 0 ? max(0, block_q0 + 1 - s.window) / 64 : 0;
     const int kt_last = block_q1 / 64;
+    const int kt0 = kt_first + group, kt_end = kt_last + group;  // the group's tiles, as in the forward
     u32x4 rk[NL], rv[NL];
-    fetch.load(kp, kt_first * 64, rk);
-    fetch.load(vp, kt_first * 64, rv);
+    fetch.load(kp, min(kt0, kt_last) * 64, rk);
+    fetch.load(vp, min(kt0, kt_last) * 64, rv);
+    if (pass == 0) {  // (both blocks of a workgroup lie in one plane)
+      float* const part = reinterpret_cast<float*>(flash_lds + 2 * ftile(D));  // the first group's second pair, still unused
+      static_assert(FT / (D / 8) * D * 4 <= 2 * ftile(D), "the sample's partial sums fit");
+      key_sample_sum<D>(kp, s.kv.rs, T, part);
+      __syncthreads();
+      if (threadIdx.x < D) {
+        float total = 0.0f;
+#pragma unroll
+        for (int r = 0; r < FT / (D / 8); ++r) total += part[r * D + threadIdx.x];
+        mean_key[threadIdx.x] = total / static_cast<float>(min(T, 64));
+      }
+    }
     __syncthreads();  // the previous pass's reads of the first pair are done
-    tile_store_rows<D>(smem, rk);
-    tile_store_rows<D>(smem + ftile(D), rv);
-    if (kt_first < kt_last) {
-      fetch.load(kp, kt_first * 64 + 64, rk);
-      fetch.load(vp, kt_first * 64 + 64, rv);
+    tile_store_rows<D, NT>(smem, rk);
+    tile_store_rows<D, NT>(smem + ftile(D), rv);
+    if (kt0 + GROUPS <= kt_last) {
+      fetch.load(kp, (kt0 + GROUPS) * 64, rk);
+      fetch.load(vp, (kt0 + GROUPS) * 64, rv);
     }
     // The tile pipeline and the split into unmasked tiles, the wave's diagonal tile and the other
     // waves' tiles are the forward kernel's.
     const char* k_rows;
     const char* v_rows;
     auto advance = [&](int kt) {
-      const int cur = (kt - kt_first) & 1;
+      const int cur = GROUPS == 1 ? (kt - kt_first) & 1 : (kt - kt0) / GROUPS & 1;
       k_rows = smem + cur * 2 * ftile(D);
       v_rows = k_rows + ftile(D);
       __syncthreads();  // this pair is complete, and every wave is done with the other one
-      if (kt < kt_last) {
+      if (kt + GROUPS <= kt_last) {
         char* next = smem + (cur ^ 1) * 2 * ftile(D);
-        tile_store_rows<D>(next, rk);
-        tile_store_rows<D>(next + ftile(D), rv);
-        if (kt + 1 < kt_last) {
-          fetch.load(kp, kt * 64 + 128, rk);
-          fetch.load(vp, kt * 64 + 128, rv);
+        tile_store_rows<D, NT>(next, rk);
+        tile_store_rows<D, NT>(next + ftile(D), rv);
+        if (kt + 2 * GROUPS <= kt_last) {
+          fetch.load(kp, (kt + 2 * GROUPS) * 64, rk);
+          fetch.load(vp, (kt + 2 * GROUPS) * 64, rv);
         }
       }
     };
-    int kt = kt_first;
+    int kt = kt0;
     if constexpr (WIN) {
-      for (; kt <= kt_last; ++kt) {
+      for (; kt <= kt_end; kt += GROUPS) {
         advance(kt);
         const int key0 = kt * 64;
-        if (key0 <= wave_q0 + 31 && key0 + 63 + s.window > wave_q0)
+        if ((GROUPS == 1 || kt <= kt_last) && key0 <= wave_q0 + 31 && key0 + 63 + s.window > wave_q0)
           flash_dq_tile<D, true>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, key0, q_row, T, s.window,
                                  lane);
       }
     } else if (wave_q0 < T) {
       const int diag_kt = wave_q0 / 64;
-      for (; kt < diag_kt; ++kt) {
+      for (; kt < diag_kt; kt += GROUPS) {
         advance(kt);
         flash_dq_tile<D, false>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, kt * 64, q_row, T, 0, lane);
       }
-      advance(kt);
-      flash_dq_tile<D, true>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, kt * 64, q_row, T, 0, lane);
-      ++kt;
+      if (GROUPS == 1 || kt == diag_kt) {
+        advance(kt);
+        flash_dq_tile<D, true>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, kt * 64, q_row, T, 0, lane);
+        kt += GROUPS;
+      }
     }
-    for (; kt <= kt_last; ++kt) advance(kt);  // tiles of the block's later waves (same barrier count for all)
+    for (; kt <= kt_end; kt += GROUPS) advance(kt);  // tiles of the block's later waves (same barrier count for all)
+    if constexpr (GROUPS > 1) {
+      constexpr int PART = (MT * 16 + 1) * 64;
+      float* const meet = reinterpret_cast<float*>(flash_lds);
+      __syncthreads();  // every wave is done with the tiles
+      if (group > 0) {
+        float* mine = meet + ((group - 1) * ROW_WAVES + wave) * PART + lane;
+        mine[0] = ds_sum;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int vv = 0; vv < 16; ++vv) mine[(1 + mt * 16 + vv) * 64] = dq[mt][vv];
+      }
+      __syncthreads();
+      if (group > 0) return;
+#pragma unroll
+      for (int g = 0; g < GROUPS - 1; ++g) {
+        const float* part = meet + (g * ROW_WAVES + wave) * PART + lane;
+        ds_sum += part[0];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int vv = 0; vv < 16; ++vv) dq[mt][vv] += part[(1 + mt * 16 + vv) * 64];
+      }
+    }
     {
-      const float* mean = key_mean + (static_cast<long>(b) * s.kv_heads + kvh) * D;
       const float row_sum = halves_sum(ds_sum);  // the two half-waves hold half the keys each
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
-          const float4 m = *reinterpret_cast<const float4*>(mean + mt * 32 + 8 * q4 + 4 * lg);
+          const float4 m = *reinterpret_cast<const float4*>(mean_key + mt * 32 + 8 * q4 + 4 * lg);
           dq[mt][4 * q4 + 0] = fmaf(-row_sum, m.x, dq[mt][4 * q4 + 0]);
           dq[mt][4 * q4 + 1] = fmaf(-row_sum, m.y, dq[mt][4 * q4 + 1]);
           dq[mt][4 * q4 + 2] = fmaf(-row_sum, m.z, dq[mt][4 * q4 + 2]);
@@ -997,10 +1144,46 @@ FlashShape make_shape(uint64_t batch, uint64_t heads, uint64_t kv_heads, uint64_
 // (forward 43.2 -> 42.1 us at 768 pairs). `also_rounds`: also when the pairs need more than one
 // round, whose last would run part empty (the blocks go out heaviest first).
 int flash_single(omx_ctx* ctx, unsigned pair_groups, int per_cu, bool also_rounds) {
-  if (ctx->flash_schedule != 0) return ctx->flash_schedule == 1 ? 1 : 0;  // forced (tests cover both)
+  if (ctx->flash_schedule != 0) return ctx->flash_schedule == 2 ? 0 : 1;  // forced (tests cover both)
   const unsigned places = static_cast<unsigned>(ctx->cu_count > 0 ? ctx->cu_count : 256) * per_cu;
   if (pair_groups <= places) return 1;
   return also_rounds ? 1 : 0;
+}
+
+// f(integral_constant) of a group count the kernels of head dim D are compiled for.
+template <int D, typename F>
+void for_groups(int groups, F&& f) {
+  if (groups == 1) return f(std::integral_constant<int, 1>{});
+  if constexpr (D == 64) {
+    if (groups == 4) return f(std::integral_constant<int, 4>{});
+  }
+  f(std::integral_constant<int, 2>{});
+}
+
+// How many groups of waves share the 64-row tiles that a row block walks (`tiles`: the most of them; `planes` of `time` rows).
+// A block's tiles are a chain, 0.9 us each where a wave has its SIMD to itself, and a causal block's neighbours are done
+// before the heaviest one. Two groups of 64 rows a workgroup halve the chain and double the workgroups, four of 32 rows do
+// so again, while the chip has places for them: the groups' tiles take 72 and 144 KiB of LDS (two and one workgroups per
+// compute unit, at head_dim 128 one), and a tile serves 64 or 32 rows instead of 128, so a full chip loses by them (batch 16
+// of 12 heads x 1024: 47 -> 62 us). Where the places are taken once over, the chains' skew still pays for a round or so more.
+// us with 1 / 2 / 4 groups, forward: 12 heads x 2048: 33 / 24 / 33; 8 x 1024: 18.5 / 13.2 / 11.2; 7 x 8 x 500: 12.2 / 10.5 / 23;
+// 96 x 360: 11.8 / 13.6 / 33; backward of 8 heads over 2 key heads x 777, batch 2: 114 / 72 / 63. Over 187 shapes (558 passes) the rule
+// is 0.5 % behind the best count on average, 12 % ahead of one group.
+int flash_groups(omx_ctx* ctx, unsigned planes, int time, int tiles, bool window, int dim) {
+  const int most = dim == 64 ? 4 : 2;
+  if (ctx->flash_schedule >= 3) return std::min(most, ctx->flash_schedule == 3 ? 2 : 4);  // forced
+  if (ctx->flash_schedule != 0 || tiles < 2) return 1;
+  const long units = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const long two = static_cast<long>(planes) * ((time + 63) / 64), four = static_cast<long>(planes) * ((time + 31) / 32);
+  const int skew = window ? 0 : tiles;
+  if (dim == 128) return two <= units || (two <= 2 * units && skew >= 12) ? 2 : 1;
+  if ((four <= units && tiles >= 4) || (four <= 2 * units && skew >= 24)) return 4;
+  return two <= 2 * units || (two <= 3 * units && skew >= 12) || (two <= 4 * units && skew >= 32) ? 2 : 1;
+}
+
+// The most 64-row tiles that a 128-row block walks.
+int flash_tiles(const FlashShape& s) {
+  return ((s.window > 0 && s.window < s.time - 127 ? s.window + 127 : s.time) + 63) / 64;
 }
 
 template <int D>
@@ -1010,8 +1193,11 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
   // Two 128-row query blocks per workgroup (see the kernel), or one when the pairs would not fill
   // the chip's workgroup places.
   const unsigned q_blocks = static_cast<unsigned>((s.time + 127) / 128), planes = static_cast<unsigned>(s.batch * s.heads);
-  s.q_single = flash_single(ctx, (q_blocks + 1) / 2 * planes, D == 64 ? 3 : 2, false);
-  dim3 grid((s.q_single ? q_blocks : (q_blocks + 1) / 2) * planes), block(FT);
+  const int tiles = flash_tiles(s);
+  const int groups = flash_groups(ctx, planes, s.time, tiles, s.window > 0, D);
+  s.q_single = groups > 1 || flash_single(ctx, (q_blocks + 1) / 2 * planes, D == 64 ? 3 : 2, false);
+  const unsigned rows = 128 / groups;
+  dim3 grid((s.q_single ? (s.time + rows - 1) / rows : (q_blocks + 1) / 2) * planes), block(FT);
   // Causal-counted work: half of the 4 B H T^2 D of the two full products.
   OmxKernelTimer timer(ctx, OMX_K_FLASH_FWD, 2.0 * s.batch * s.heads * static_cast<double>(s.time) * s.time * D);
   auto go = [&](auto kernel, auto* out_ptr, unsigned short* resid_ptr) {
@@ -1019,56 +1205,64 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
                      ctx->fault, tag);
   };
   unsigned short* resid = static_cast<unsigned short*>(out_residual);
-  if (out_dtype == OMX_BF16) {
-    if (s.window > 0) go(flash_fwd_kernel<D, unsigned short, true>, static_cast<unsigned short*>(out), resid);
-    else go(flash_fwd_kernel<D, unsigned short, false>, static_cast<unsigned short*>(out), resid);
-  } else {
-    if (s.window > 0) go(flash_fwd_kernel<D, float, true>, static_cast<float*>(out), static_cast<unsigned short*>(nullptr));
-    else go(flash_fwd_kernel<D, float, false>, static_cast<float*>(out), static_cast<unsigned short*>(nullptr));
-  }
+  auto with_groups = [&](auto count) {
+    constexpr int G = decltype(count)::value;
+    if (out_dtype == OMX_BF16) {
+      if (s.window > 0) go(flash_fwd_kernel<D, unsigned short, true, G>, static_cast<unsigned short*>(out), resid);
+      else go(flash_fwd_kernel<D, unsigned short, false, G>, static_cast<unsigned short*>(out), resid);
+    } else {
+      if (s.window > 0) go(flash_fwd_kernel<D, float, true, G>, static_cast<float*>(out), static_cast<unsigned short*>(nullptr));
+      else go(flash_fwd_kernel<D, float, false, G>, static_cast<float*>(out), static_cast<unsigned short*>(nullptr));
+    }
+  };
+  for_groups<D>(groups, with_groups);
 }
 
 template <int D>
 void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short* k, const unsigned short* v,
                      const unsigned short* out, const unsigned short* resid, const float* lse, float* delta,
-                     float* key_mean, const unsigned short* gy, void* gq, void* gk, void* gv, int32_t grad_dtype,
+                     const unsigned short* gy, void* gq, void* gk, void* gv, int32_t grad_dtype,
                      const FlashShape& shape, unsigned long long tag) {
   FlashShape s = shape;
   // Five causal-counted products (S and dP twice each way, dV, dQ, dK) of B H T^2 D each.
   OmxKernelTimer timer(ctx, OMX_K_FLASH_BWD, 5.0 * s.batch * s.heads * static_cast<double>(s.time) * s.time * D);
-  omx_launch_timed(ctx, flash_key_mean_kernel<D>, dim3(static_cast<unsigned>(s.batch * s.kv_heads)), dim3(256), 0,
-                   timer.start(), nullptr, k, key_mean, s);
   // dQ first: it also leaves delta = dO . O per row for the dK/dV pass.
   dim3 block(FT);
   const unsigned pairs = static_cast<unsigned>((s.time + 127) / 128 + 1) / 2;  // two 128-row blocks per workgroup
   const unsigned blocks = static_cast<unsigned>((s.time + 127) / 128);
   const unsigned kv_planes = static_cast<unsigned>(s.batch * s.kv_heads), q_planes = static_cast<unsigned>(s.batch * s.heads);
-  s.q_single = flash_single(ctx, pairs * q_planes, D == 64 ? 3 : 2, false);
-  s.kv_single = flash_single(ctx, pairs * kv_planes, 2, true);
-  dim3 kv_grid((s.kv_single ? blocks : pairs) * kv_planes);
-  dim3 q_grid((s.q_single ? blocks : pairs) * q_planes);
-  auto go = [&](auto dq_kernel, auto dkv_kernel, auto* gq_ptr, auto* gk_ptr, auto* gv_ptr) {
-    omx_launch(ctx, dq_kernel, q_grid, block, 0, q, k, v, out, resid, lse, delta, key_mean, gy, gq_ptr, s,
-                       ctx->fault, tag);
-    omx_launch_timed(ctx, dkv_kernel, kv_grid, block, 0, nullptr, timer.stop(), q, k, v, lse, delta, gy, gk_ptr, gv_ptr, s,
+  const int tiles = flash_tiles(s);
+  const int q_groups = flash_groups(ctx, q_planes, s.time, tiles, s.window > 0, D);
+  const int kv_groups = flash_groups(ctx, kv_planes, s.time, static_cast<int>(std::min<long>(static_cast<long>(tiles) * s.rep, 1 << 20)), s.window > 0, D);
+  const unsigned q_rows = 128 / q_groups, kv_rows = 128 / kv_groups;
+  s.q_single = q_groups > 1 || flash_single(ctx, pairs * q_planes, D == 64 ? 3 : 2, false);
+  s.kv_single = kv_groups > 1 || flash_single(ctx, pairs * kv_planes, 2, true);
+  dim3 kv_grid((s.kv_single ? (s.time + kv_rows - 1) / kv_rows : pairs) * kv_planes);
+  dim3 q_grid((s.q_single ? (s.time + q_rows - 1) / q_rows : pairs) * q_planes);
+  auto go_dq = [&](auto kernel, auto* gq_ptr) {
+    omx_launch_timed(ctx, kernel, q_grid, block, 0, timer.start(), nullptr, q, k, v, out, resid, lse, delta, gy, gq_ptr, s, ctx->fault, tag);
+  };
+  auto go_dkv = [&](auto kernel, auto* gk_ptr, auto* gv_ptr) {
+    omx_launch_timed(ctx, kernel, kv_grid, block, 0, nullptr, timer.stop(), q, k, v, lse, delta, gy, gk_ptr, gv_ptr, s,
                      ctx->fault, tag);
   };
-  if (grad_dtype == OMX_BF16) {
-    typedef unsigned short T16;
-    if (s.window > 0)
-      go(flash_bwd_dq_kernel<D, T16, true>, flash_bwd_dkv_kernel<D, T16, true>, static_cast<T16*>(gq), static_cast<T16*>(gk),
-         static_cast<T16*>(gv));
-    else
-      go(flash_bwd_dq_kernel<D, T16, false>, flash_bwd_dkv_kernel<D, T16, false>, static_cast<T16*>(gq),
-         static_cast<T16*>(gk), static_cast<T16*>(gv));
-  } else {
-    if (s.window > 0)
-      go(flash_bwd_dq_kernel<D, float, true>, flash_bwd_dkv_kernel<D, float, true>, static_cast<float*>(gq),
-         static_cast<float*>(gk), static_cast<float*>(gv));
-    else
-      go(flash_bwd_dq_kernel<D, float, false>, flash_bwd_dkv_kernel<D, float, false>, static_cast<float*>(gq),
-         static_cast<float*>(gk), static_cast<float*>(gv));
-  }
+  auto both = [&](auto* gq_ptr, auto* gk_ptr, auto* gv_ptr) {
+    typedef std::remove_pointer_t<decltype(gq_ptr)> T;
+    for_groups<D>(q_groups, [&](auto count) {
+      constexpr int G = decltype(count)::value;
+      if (s.window > 0) go_dq(flash_bwd_dq_kernel<D, T, true, G>, gq_ptr);
+      else go_dq(flash_bwd_dq_kernel<D, T, false, G>, gq_ptr);
+    });
+    for_groups<D>(kv_groups, [&](auto count) {
+      constexpr int G = decltype(count)::value;
+      if (s.window > 0) go_dkv(flash_bwd_dkv_kernel<D, T, true, G>, gk_ptr, gv_ptr);
+      else go_dkv(flash_bwd_dkv_kernel<D, T, false, G>, gk_ptr, gv_ptr);
+    });
+  };
+  if (grad_dtype == OMX_BF16)
+    both(static_cast<unsigned short*>(gq), static_cast<unsigned short*>(gk), static_cast<unsigned short*>(gv));
+  else
+    both(static_cast<float*>(gq), static_cast<float*>(gk), static_cast<float*>(gv));
 }
 
 // The tile loads add a thread's rows as a 32-bit byte offset to a scalar base.
@@ -1115,19 +1309,17 @@ int32_t omx_flash_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, cons
   if (int32_t rc = check_row_strides(ctx, s); rc != OMX_OK) return rc;
   const long rows = static_cast<long>(batch * heads * time);
   void* ws = nullptr;
-  const long rows4 = (rows + 3) & ~3L;  // the mean key rows are read four values at a time
-  int32_t rc = omx_workspace(ctx, (rows4 + static_cast<long>(batch * kv_heads * dim)) * sizeof(float), &ws);
+  int32_t rc = omx_workspace(ctx, rows * sizeof(float), &ws);
   if (rc != OMX_OK) return rc;
   float* delta = static_cast<float*>(ws);
-  float* key_mean = delta + rows4;
   const unsigned short* qs = static_cast<const unsigned short*>(q);
   const unsigned short* ks = static_cast<const unsigned short*>(k);
   const unsigned short* vs = static_cast<const unsigned short*>(v);
   const unsigned short* os = static_cast<const unsigned short*>(out);
   const unsigned short* rs = static_cast<const unsigned short*>(out_residual);
   const unsigned short* gs = static_cast<const unsigned short*>(gy);
-  if (dim == 64) launch_backward<64>(ctx, qs, ks, vs, os, rs, lse, delta, key_mean, gs, gq, gk, gv, grad_dtype, s, tag);
-  else launch_backward<128>(ctx, qs, ks, vs, os, rs, lse, delta, key_mean, gs, gq, gk, gv, grad_dtype, s, tag);
+  if (dim == 64) launch_backward<64>(ctx, qs, ks, vs, os, rs, lse, delta, gs, gq, gk, gv, grad_dtype, s, tag);
+  else launch_backward<128>(ctx, qs, ks, vs, os, rs, lse, delta, gs, gq, gk, gv, grad_dtype, s, tag);
   OMX_LAUNCH_CHECK(ctx, "flash backward kernels");
   return OMX_OK;
 }

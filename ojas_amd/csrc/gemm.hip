@@ -931,7 +931,7 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value) {
     return OMX_OK;
   }
   if (name && strcmp(name, "flash_schedule") == 0) {
-    if (value < 0 || value > 2) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: flash_schedule takes 0..2");
+    if (value < 0 || value > 4) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: flash_schedule takes 0..4");
     ctx->flash_schedule = static_cast<int>(value);
     return OMX_OK;
   }

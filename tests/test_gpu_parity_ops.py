@@ -941,6 +941,30 @@ def test_causal_sdpa_bf16_mfma(be, shape, hkv, window, flash_schedule):
     close(be.download_f32(gv16), ogv, BF16_TOL, "flash gv bf16")
 
 
+@pytest.mark.parametrize("groups", [2, 4])
+@pytest.mark.parametrize("shape,hkv,window", FLASH_SHAPES + [((1, 2, 1, 64), 1, None), ((2, 3, 33, 64), 3, None), ((1, 6, 65, 64), 2, None),
+                                                             ((1, 2, 97, 128), 1, None), ((1, 4, 321, 64), 1, 40), ((1, 2, 449, 128), 2, 65)])
+def test_causal_sdpa_bf16_with_tiles_shared_by_groups_of_waves(be, shape, hkv, window, groups):
+    """The same with two and four groups of waves sharing a row block's tiles, whatever the shape: groups without a tile, waves
+    past the sequence's end, key heads whose query heads' tiles alternate between groups; then a value that is not finite
+    in a tile that a later group takes."""
+    from ojas_amd.backend import BF16, OjasError
+
+    be.set_option("flash_schedule", 3 if groups == 2 else 4)
+    try:
+        test_causal_sdpa_bf16_mfma(be, shape, hkv, window, f"{groups} groups")
+        b, h, t, d = shape
+        for at in {t - 1, min(64, t - 1)}:
+            x = np.ones((b, hkv, t, d), np.float32)
+            x[0, 0, at, 3] = np.inf
+            q, ok, bad = (be.upload(a, BF16) for a in (np.ones((b, h, t, d), np.float32), np.ones((b, hkv, t, d), np.float32), x))
+            be.causal_sdpa_forward(q, ok, bad, window, out_dtype=BF16)
+            with pytest.raises(OjasError):
+                be.sync()
+    finally:
+        be.set_option("flash_schedule", 0)
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("shared", [(0, 4, 0), (0, 0, 4), (4, 4, 4)])
 def test_causal_attention_keeps_its_accuracy_when_rows_share_a_component(be, dim, shared):
