@@ -18,14 +18,19 @@
 // moving. The other operand of that product is read from LDS along its fast index: one 16-byte read serves four
 // interleaved blocks of result columns (block c VW + e holds columns 16 VW c + VW i + e).
 //
-// 64-row tiles are fetched into registers while the previous one is multiplied. Where there are few rows the four
-// waves of a workgroup split the keys (KW = 4) instead of the rows and meet in LDS; the key / value pass splits
+// 64-row tiles are fetched into registers while the previous one is multiplied. Where there are few rows, or the other
+// side is long (at_narrow), the four waves of a workgroup split the keys (KW = 4) instead of the rows and meet in LDS: no wave
+// reads another's blocks then, so they come from memory straight into operands, a block ahead, with no barrier in the
+// loop. A block that is read in both forms (keys in the dQ pass, rows in the key / value pass) goes through 16 rows of LDS of the
+// wave's own for the second: fetched twice, the passes were bound by their loads' latency (2 x 8 heads over 2 x 777, backward:
+// 131 us through shared tiles, 118 with two fetches, 104). The key / value pass splits
 // its rows over the grid when keys alone do not fill the chip, and a second launch adds the parts in order.
 // No atomics; every sum has a fixed order.
 //
-// Before and after, us, forward / backward (batch x heads over KV heads x time x head dim): 8 x 4/4 x 256 x 64: 38 / 109 ->
-// 13 / 34; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370 -> 20 / 66; 16 x 12/12 x 512 x 64: 272 / 1337 -> 132 / 439 (48 and
-// 37 TFLOP/s, causal-counted); 1 x 2/1 x 3000 x 128: 696 / 3334 -> 151 / 409.
+// On vector instructions, through shared tiles and now, us, forward / backward (batch x heads over KV heads x time x head
+// dim): 8 x 4/4 x 256 x 64: 38 / 109, 13 / 34, 11 / 32; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370, 20 / 66, 18 / 59; 16 x 12/12
+// x 512 x 64 (shared tiles still): 272 / 1337, 132 / 439 (48 and 37 TFLOP/s, causal-counted); 1 x 2/1 x 3000 x 128: 696 / 3334, 151 /
+// 409, 89 / 237.
 #include <algorithm>
 #include <cmath>
 
@@ -42,14 +47,16 @@ __device__ __forceinline__ floatx4_a at_mfma(float a, float b, floatx4_a c) {
 }
 __device__ __forceinline__ floatx4_a at_zero() { return floatx4_a{0.0f, 0.0f, 0.0f, 0.0f}; }
 // Over the four lanes that hold one row.
-__device__ __forceinline__ float at_row_max(float v) {
-  v = fmaxf(v, __shfl_xor(v, 16));
-  return fmaxf(v, __shfl_xor(v, 32));
+// (v_permlane16_swap and v_permlane32_swap of a value with its copy leave both lanes' values in both: no LDS round trip)
+template <typename F>
+__device__ __forceinline__ float at_row(float v, F f) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-__device__ __forceinline__ float at_row_sum(float v) {
-  v += __shfl_xor(v, 16);
-  return v + __shfl_xor(v, 32);
-}
+__device__ __forceinline__ float at_row_max(float v) { return at_row(v, [](float x, float y) { return fmaxf(x, y); }); }
+__device__ __forceinline__ float at_row_sum(float v) { return at_row(v, [](float x, float y) { return x + y; }); }
 
 template <int D>
 struct AtDim {
@@ -89,6 +96,66 @@ struct AtTile {
       }
       *reinterpret_cast<float4*>(lds + r * AtDim<D>::P + 4 * c) = v;
     }
+  }
+};
+
+// ---- without LDS: a wave that shares its 16-row blocks with no other reads them straight into operands
+__device__ __forceinline__ float4 at_widen(const float4& v) { return v; }
+__device__ __forceinline__ float4 at_widen(const uint2& w) {
+  return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
+                     __uint_as_float(w.y & 0xffff0000u));
+}
+__device__ __forceinline__ float at_value(float v) { return v; }
+__device__ __forceinline__ float at_value(unsigned short v) { return dev_bf16_bits_to_f32(v); }
+// One block for at_dot: lane i's row (`row` points to it), pieces 4 g of each 16 columns.
+template <int D, typename T>
+struct AtDotBlock {
+  using Raw = std::conditional_t<sizeof(T) == 4, float4, uint2>;
+  Raw raw[AtDim<D>::S];
+  __device__ __forceinline__ void fetch(const T* row, int g) {
+#pragma unroll
+    for (int s = 0; s < AtDim<D>::S; ++s) raw[s] = *reinterpret_cast<const Raw*>(row + 16 * s + 4 * g);
+  }
+  __device__ __forceinline__ floatx4_a dot(const float4 (&own)[AtDim<D>::S]) const {
+    floatx4_a acc = at_zero();
+#pragma unroll
+    for (int s = 0; s < AtDim<D>::S; ++s) {
+      const float4 t = at_widen(raw[s]);
+      acc = at_mfma(t.x, own[s].x, acc);
+      acc = at_mfma(t.y, own[s].y, acc);
+      acc = at_mfma(t.z, own[s].z, acc);
+      acc = at_mfma(t.w, own[s].w, acc);
+    }
+    return acc;
+  }
+};
+// The block as at_accumulate reads it, in LDS of this wave's own (16 rows of pitch P).
+template <int D>
+__device__ __forceinline__ void at_stage(const AtDotBlock<D, float>& block, float* tile16, int i, int g) {
+#pragma unroll
+  for (int s = 0; s < AtDim<D>::S; ++s) *reinterpret_cast<float4*>(tile16 + i * AtDim<D>::P + 16 * s + 4 * g) = block.raw[s];
+}
+// One block for at_accumulate: rows 4 g + j (`rows[j]` point to them), columns VW i .. of each 64 (of 32, of 16).
+template <int D, typename T>
+struct AtSumBlock {
+  using X = AtDim<D>;
+  T raw[4][X::NC][X::VW];
+  template <typename F>
+  __device__ __forceinline__ void fetch(F row_at, int i) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const T* row = row_at(j) + X::VW * i;
+#pragma unroll
+      for (int c = 0; c < X::NC; ++c) __builtin_memcpy(raw[j][c], __builtin_assume_aligned(row + 64 * c, X::VW * sizeof(T)), X::VW * sizeof(T));
+    }
+  }
+  __device__ __forceinline__ void accumulate(const floatx4_a& weight, floatx4_a (&out)[X::S]) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c = 0; c < X::NC; ++c)
+#pragma unroll
+        for (int e = 0; e < X::VW; ++e) out[c * X::VW + e] = at_mfma(at_value(raw[j][c][e]), weight[j], out[c * X::VW + e]);
   }
 };
 
@@ -193,11 +260,12 @@ __device__ __forceinline__ void at_own(const float* row, float4 (&own)[AtDim<D>:
 template <int D, int KW, typename TK>
 __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   using X = AtDim<D>;
-  constexpr int QW = 4 / KW, BQ = 16 * QW, NB = AT_ROWS / 16 / KW;
-  __shared__ __align__(16) float lds[2 * AT_ROWS * X::P];
+  // KW = 4: nothing but the waves' sums goes through LDS, and the keys go round in blocks of 16 BLOCKS.
+  constexpr int QW = 4 / KW, BQ = 16 * QW, BLOCKS = KW == 1 ? 4 : D <= 64 ? 2 : 1, KEYS = 16 * BLOCKS;
+  __shared__ __align__(16) float lds[KW == 1 ? 2 * AT_ROWS * X::P : 128 + 4 * X::S * 256];
   float* kt = lds;
   float* vt = lds + AT_ROWS * X::P;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int qw = wave % QW, kw = wave / QW;
   const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
   const int rows = a.tq * a.rep;
@@ -211,21 +279,14 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   const int low = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
   const int first_pos = a.q_pos0 + at_unpack(r0, a.rep).query;
   const int last_pos = a.q_pos0 + at_unpack(min(r0 + BQ, rows) - 1, a.rep).query;
-  int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / AT_ROWS, t_last = last_pos / AT_ROWS;
+  int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / KEYS, t_last = last_pos / KEYS;
   at_key_part(a, &t_first, &t_last);
   const TK* kb = static_cast<const TK*>(a.k) + b * a.k_b + kvh * a.k_h;
   const TK* vb = static_cast<const TK*>(a.v) + b * a.k_b + kvh * a.k_h;
-  AtTile<D, TK> kn, vn;
-  auto fetch = [&](int t) {
-    auto row_of = [&](const TK* base, int row) {
-      const int key = t * AT_ROWS + row;
-      // A ring wraps at most once over the keys that are read (slot0 + key can pass 2^31).
-      unsigned int slot = static_cast<unsigned int>(a.slot0) + key;
-      slot = slot >= static_cast<unsigned int>(a.capacity) ? slot - a.capacity : slot;
-      return key < a.tk ? base + static_cast<long>(slot) * a.k_t : nullptr;
-    };
-    kn.fetch([&](int row) { return row_of(kb, row); });
-    vn.fetch([&](int row) { return row_of(vb, row); });
+  auto slot_at = [&](int key) {
+    // A ring wraps at most once over the keys that are read (slot0 + key can pass 2^31).
+    const unsigned int slot = static_cast<unsigned int>(a.slot0) + key, capacity = a.capacity;
+    return static_cast<long>(slot >= capacity ? slot - capacity : slot) * a.k_t;
   };
   const float scale2 = a.scale * AT_LOG2E;
   floatx4_a o[X::S];
@@ -233,29 +294,20 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   for (int m = 0; m < X::S; ++m) o[m] = at_zero();
   float mx = -INFINITY, sum = 0.0f;  // in the exp2 domain; `sum` over this lane's keys only
   bool bad = false;
-  if (t_first <= t_last) fetch(t_first);
-  for (int t = t_first; t <= t_last; ++t) {
-    __syncthreads();  // the previous tile has been read
-    kn.store(kt);
-    vn.store(vt);
-    __syncthreads();
-    if (t < t_last) fetch(t + 1);
-    floatx4_a s[NB];
+  // Scores to weights for `key0` and the keys after it: masks, the running maximum, the rescaling that it asks for.
+  auto weights = [&](floatx4_a (&s)[BLOCKS], int key0) {
     float top = -INFINITY;
 #pragma unroll
-    for (int n = 0; n < NB; ++n) {
-      const int row = (kw * NB + n) * 16;
-      s[n] = at_dot<D>(kt + row * X::P, q, i, g);
+    for (int n = 0; n < BLOCKS; ++n)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int key = t * AT_ROWS + row + 4 * g + v;
+        const int key = key0 + n * 16 + 4 * g + v;
         const bool seen = key <= pos && key >= low;
         const float x = s[n][v] * scale2;
         bad |= seen && !dev_finite(x);
         s[n][v] = seen ? x : -INFINITY;
         top = fmaxf(top, s[n][v]);
       }
-    }
     top = at_row_max(top);
     const float mx_new = fmaxf(mx, top), base = mx_new == -INFINITY ? 0.0f : mx_new;
     const float rescale = __builtin_amdgcn_exp2f(mx - base);  // 0 on the first keys; 1 when none were seen yet: the sums are 0
@@ -266,13 +318,59 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) o[m][v] *= rescale;
 #pragma unroll
-    for (int n = 0; n < NB; ++n) {
+    for (int n = 0; n < BLOCKS; ++n)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         s[n][v] = __builtin_amdgcn_exp2f(s[n][v] - base);
         sum += s[n][v];
       }
-      at_accumulate<D>(vt + (kw * NB + n) * 16 * X::P, s[n], o, i, g);
+  };
+  if constexpr (KW == 1) {
+    AtTile<D, TK> kn, vn;
+    auto fetch = [&](int t) {
+      auto row_of = [&](const TK* base, int row) {
+        const int key = t * AT_ROWS + row;
+        return key < a.tk ? base + slot_at(key) : nullptr;
+      };
+      kn.fetch([&](int row) { return row_of(kb, row); });
+      vn.fetch([&](int row) { return row_of(vb, row); });
+    };
+    if (t_first <= t_last) fetch(t_first);
+    for (int t = t_first; t <= t_last; ++t) {
+      __syncthreads();  // the previous tile has been read
+      kn.store(kt);
+      vn.store(vt);
+      __syncthreads();
+      if (t < t_last) fetch(t + 1);
+      floatx4_a s[BLOCKS];
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n) s[n] = at_dot<D>(kt + n * 16 * X::P, q, i, g);
+      weights(s, t * KEYS);
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n) at_accumulate<D>(vt + n * 16 * X::P, s[n], o, i, g);
+    }
+  } else {
+    // Values are on their way while the scores are formed, the next keys during softmax and the second product. (Keys past
+    // the last one are read from it; their weights are 0.)
+    AtDotBlock<D, TK> keys[BLOCKS];
+    AtSumBlock<D, TK> values[BLOCKS];
+    auto fetch = [&](int t) {
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n) keys[n].fetch(kb + slot_at(min(t * KEYS + n * 16 + i, a.tk - 1)), g);
+    };
+    int t = t_first + kw;
+    if (t <= t_last) fetch(t);
+    for (; t <= t_last; t += KW) {
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n)
+        values[n].fetch([&](int j) { return vb + slot_at(min(t * KEYS + n * 16 + 4 * g + j, a.tk - 1)); }, i);
+      floatx4_a s[BLOCKS];
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n) s[n] = keys[n].dot(q);
+      fetch(min(t + KW, t_last));
+      weights(s, t * KEYS);
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n) values[n].accumulate(s[n], o);
     }
   }
   sum = at_row_sum(sum);
@@ -617,11 +715,12 @@ struct AtGrad {
 template <int D, int KW>
 __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
   using X = AtDim<D>;
-  constexpr int QW = 4 / KW, BQ = 16 * QW, NB = AT_ROWS / 16 / KW;
-  __shared__ __align__(16) float lds[2 * AT_ROWS * X::P];
+  constexpr int QW = 4 / KW, BQ = 16 * QW, BLOCKS = KW == 1 ? 4 : 1, KEYS = 16 * BLOCKS;
+  __shared__ __align__(16) float lds[KW == 1 ? 2 * AT_ROWS * X::P : 4 * 16 * X::P];
+  static_assert(16 * X::P >= X::S * 256, "the waves' sums fit");
   float* kt = lds;
   float* vt = lds + AT_ROWS * X::P;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int qw = wave % QW, kw = wave / QW;
   const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
   const int rows = a.tq * a.rep;
@@ -652,40 +751,71 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
   const int pos = r < rows ? at.query : -1;
   const int low = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
   const int first_pos = at_unpack(r0, a.rep).query, last_pos = at_unpack(min(r0 + BQ, rows) - 1, a.rep).query;
-  const int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / AT_ROWS, t_last = last_pos / AT_ROWS;
+  const int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / KEYS, t_last = last_pos / KEYS;
   const float* kb = static_cast<const float*>(a.k) + b * a.k_b + kvh * a.k_h;
   const float* vb = static_cast<const float*>(a.v) + b * a.k_b + kvh * a.k_h;
-  AtTile<D, float> kn, vn;
-  auto fetch = [&](int t) {
-    kn.fetch([&](int row) { const int key = t * AT_ROWS + row; return key < a.tk ? kb + static_cast<long>(key) * a.k_t : nullptr; });
-    vn.fetch([&](int row) { const int key = t * AT_ROWS + row; return key < a.tk ? vb + static_cast<long>(key) * a.k_t : nullptr; });
-  };
   const AtGrad grad{a.scale, a.scale * AT_LOG2E};
   floatx4_a dq[X::S];
 #pragma unroll
   for (int m = 0; m < X::S; ++m) dq[m] = at_zero();
   bool bad = false;
-  fetch(t_first);
-  for (int t = t_first; t <= t_last; ++t) {
-    __syncthreads();
-    kn.store(kt);
-    vn.store(vt);
-    __syncthreads();
-    if (t < t_last) fetch(t + 1);
+  // dS of keys key0 + 4 g + v, from the scores and dP.
+  auto slopes = [&](const floatx4_a& s, const floatx4_a& dp, int key0) {
+    floatx4_a ds;
 #pragma unroll
-    for (int n = 0; n < NB; ++n) {
-      const int row = (kw * NB + n) * 16;
-      const floatx4_a s = at_dot<D>(kt + row * X::P, q, i, g);
-      const floatx4_a dp = at_dot<D>(vt + row * X::P, dout, i, g);
-      floatx4_a ds;
+    for (int v = 0; v < 4; ++v) {
+      const int key = key0 + 4 * g + v;
+      float p, d;
+      grad(key <= pos && key >= low, s[v], dp[v], lse2, delta, &p, &d, &bad);
+      ds[v] = d;
+    }
+    return ds;
+  };
+  if constexpr (KW == 1) {
+    AtTile<D, float> kn, vn;
+    auto fetch = [&](int t) {
+      kn.fetch([&](int row) { const int key = t * AT_ROWS + row; return key < a.tk ? kb + static_cast<long>(key) * a.k_t : nullptr; });
+      vn.fetch([&](int row) { const int key = t * AT_ROWS + row; return key < a.tk ? vb + static_cast<long>(key) * a.k_t : nullptr; });
+    };
+    fetch(t_first);
+    for (int t = t_first; t <= t_last; ++t) {
+      __syncthreads();
+      kn.store(kt);
+      vn.store(vt);
+      __syncthreads();
+      if (t < t_last) fetch(t + 1);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int key = t * AT_ROWS + row + 4 * g + v;
-        float p, d;
-        grad(key <= pos && key >= low, s[v], dp[v], lse2, delta, &p, &d, &bad);
-        ds[v] = d;
+      for (int n = 0; n < BLOCKS; ++n) {
+        const int row = n * 16;
+        const floatx4_a s = at_dot<D>(kt + row * X::P, q, i, g);
+        const floatx4_a dp = at_dot<D>(vt + row * X::P, dout, i, g);
+        at_accumulate<D>(kt + row * X::P, slopes(s, dp, t * AT_ROWS + row), dq, i, g);
       }
-      at_accumulate<D>(kt + row * X::P, ds, dq, i, g);
+    }
+  } else {
+    // Keys and values come straight into the first two products' operands, a whole block ahead; the keys' other form goes through
+    // LDS of the wave's own. (Keys past the last one are read from it; their dS is 0.)
+    AtDotBlock<D, float> keys[2], values[2];
+    float* const own = lds + kw * (16 * X::P);
+    auto fetch = [&](int set, int t) {
+      const long at_key = static_cast<long>(min(t * KEYS + i, a.tk - 1)) * a.k_t;
+      keys[set].fetch(kb + at_key, g);
+      values[set].fetch(vb + at_key, g);
+    };
+    auto step = [&](int set, int t) {
+      __builtin_amdgcn_wave_barrier();  // the previous block has been read
+      at_stage<D>(keys[set], own, i, g);
+      __builtin_amdgcn_wave_barrier();
+      fetch(set ^ 1, min(t + KW, t_last));
+      const floatx4_a s = keys[set].dot(q), dp = values[set].dot(dout);
+      at_accumulate<D>(own, slopes(s, dp, t * KEYS), dq, i, g);
+    };
+    int t = t_first + kw;
+    if (t <= t_last) fetch(0, t);
+    for (; t <= t_last; t += 2 * KW) {
+      step(0, t);
+      if (t + KW > t_last) break;
+      step(1, t + KW);
     }
   }
   float* out = a.gq + q_at;
@@ -715,13 +845,14 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
 template <int D, int RW>  // RW waves share a tile's rows, 4 / RW take 16 keys each
 __global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
   using X = AtDim<D>;
-  constexpr int KG = 4 / RW, BK = 16 * KG, NB = AT_ROWS / 16 / RW;
-  __shared__ __align__(16) float lds[2 * AT_ROWS * X::P + 2 * AT_ROWS];
+  // RW = 4: nothing but the waves' sums goes through LDS; row tiles are blocks of 16 rows.
+  constexpr int KG = 4 / RW, BK = 16 * KG, NB = AT_ROWS / 16, ROWS = RW == 1 ? AT_ROWS : 16;
+  __shared__ __align__(16) float lds[RW == 1 ? 2 * AT_ROWS * X::P + 2 * AT_ROWS : 4 * 2 * 16 * X::P];
   float* qt = lds;
   float* gt = lds + AT_ROWS * X::P;
   float* lse_t = gt + AT_ROWS * X::P;
   float* delta_t = lse_t + AT_ROWS;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int kg = wave % KG, rw = wave / KG;
   const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
   const int rows = a.tq * a.rep;
@@ -733,64 +864,146 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
   // Queries that see key j: j .. min(T - 1, j + window - 1). Row tiles from the first key's to the last key's.
   const int key_last = min(j0 + BK, a.tk) - 1;
   const int q_last = a.window > 0 ? min(a.tk - 1, key_last + a.window - 1) : a.tk - 1;
-  const int u_first = j0 * a.rep / AT_ROWS, u_end = ((q_last + 1) * a.rep + AT_ROWS - 1) / AT_ROWS;
+  const int u_first = j0 * a.rep / ROWS, u_end = ((q_last + 1) * a.rep + ROWS - 1) / ROWS;
   const int share = (u_end - u_first + gridDim.z - 1) / gridDim.z;
   const int u0 = u_first + blockIdx.z * share, u1 = min(u_end, u0 + share);
   const long stat_b = (static_cast<long>(b) * a.kv_heads + kvh) * a.rep;
-  AtTile<D, float> qn, gn;
-  float lse_n = 0.0f, delta_n = 0.0f;
-  auto fetch = [&](int u) {
-    auto row_of = [&](int row, long h_stride, long t_stride) {
-      const AtRow x = at_unpack(u * AT_ROWS + row, a.rep);
-      return x.head * h_stride + static_cast<long>(x.query) * t_stride;
-    };
-    const float* qb = a.q + b * a.q_b + static_cast<long>(kvh) * a.rep * a.q_h;
-    const float* gb = a.gy + b * a.o_b + static_cast<long>(kvh) * a.rep * a.o_h;
-    qn.fetch([&](int row) { return u * AT_ROWS + row < rows ? qb + row_of(row, a.q_h, a.q_t) : nullptr; });
-    gn.fetch([&](int row) { return u * AT_ROWS + row < rows ? gb + row_of(row, a.o_h, a.o_t) : nullptr; });
-    if (threadIdx.x < AT_ROWS && u * AT_ROWS + static_cast<int>(threadIdx.x) < rows) {
-      const AtRow x = at_unpack(u * AT_ROWS + threadIdx.x, a.rep);
-      const long at = (stat_b + x.head) * a.tq + x.query;
-      lse_n = a.lse[at] * AT_LOG2E;
-      delta_n = a.delta[at];
-    }
-  };
+  const float* qb = a.q + b * a.q_b + static_cast<long>(kvh) * a.rep * a.q_h;
+  const float* gb = a.gy + b * a.o_b + static_cast<long>(kvh) * a.rep * a.o_h;
   const AtGrad grad{a.scale, a.scale * AT_LOG2E};
   floatx4_a dk[X::S], dv[X::S];
 #pragma unroll
   for (int m = 0; m < X::S; ++m) dk[m] = dv[m] = at_zero();
   bool bad = false;
-  if (u0 < u1) fetch(u0);
-  for (int u = u0; u < u1; ++u) {
-    __syncthreads();
-    qn.store(qt);
-    gn.store(gt);
-    if (threadIdx.x < AT_ROWS) {
-      lse_t[threadIdx.x] = lse_n;
-      delta_t[threadIdx.x] = delta_n;
-    }
-    __syncthreads();
-    if (u + 1 < u1) fetch(u + 1);
+  if constexpr (RW == 1) {
+    AtTile<D, float> qn, gn;
+    float lse_n = 0.0f, delta_n = 0.0f;
+    auto fetch = [&](int u) {
+      auto row_of = [&](int row, long h_stride, long t_stride) {
+        const AtRow x = at_unpack(u * AT_ROWS + row, a.rep);
+        return x.head * h_stride + static_cast<long>(x.query) * t_stride;
+      };
+      qn.fetch([&](int row) { return u * AT_ROWS + row < rows ? qb + row_of(row, a.q_h, a.q_t) : nullptr; });
+      gn.fetch([&](int row) { return u * AT_ROWS + row < rows ? gb + row_of(row, a.o_h, a.o_t) : nullptr; });
+      if (threadIdx.x < AT_ROWS && u * AT_ROWS + static_cast<int>(threadIdx.x) < rows) {
+        const AtRow x = at_unpack(u * AT_ROWS + threadIdx.x, a.rep);
+        const long at = (stat_b + x.head) * a.tq + x.query;
+        lse_n = a.lse[at] * AT_LOG2E;
+        delta_n = a.delta[at];
+      }
+    };
+    if (u0 < u1) fetch(u0);
+    for (int u = u0; u < u1; ++u) {
+      __syncthreads();
+      qn.store(qt);
+      gn.store(gt);
+      if (threadIdx.x < AT_ROWS) {
+        lse_t[threadIdx.x] = lse_n;
+        delta_t[threadIdx.x] = delta_n;
+      }
+      __syncthreads();
+      if (u + 1 < u1) fetch(u + 1);
 #pragma unroll
-    for (int n = 0; n < NB; ++n) {
-      const int row = (rw * NB + n) * 16;
-      const floatx4_a s = at_dot<D>(qt + row * X::P, k, i, g);
-      const floatx4_a dp = at_dot<D>(gt + row * X::P, v4, i, g);
-      const float4 l4 = *reinterpret_cast<const float4*>(lse_t + row + 4 * g);
-      const float4 d4 = *reinterpret_cast<const float4*>(delta_t + row + 4 * g);
-      const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
+      for (int n = 0; n < NB; ++n) {
+        const int row = n * 16;
+        const floatx4_a s = at_dot<D>(qt + row * X::P, k, i, g);
+        const floatx4_a dp = at_dot<D>(gt + row * X::P, v4, i, g);
+        const float4 l4 = *reinterpret_cast<const float4*>(lse_t + row + 4 * g);
+        const float4 d4 = *reinterpret_cast<const float4*>(delta_t + row + 4 * g);
+        const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
+        floatx4_a p, ds;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int packed = u * AT_ROWS + row + 4 * g + v, query = at_unpack(packed, a.rep).query;
+          const bool seen = packed < rows && key < a.tk && key <= query && (a.window == 0 || query < key + a.window);
+          float pv, dsv;
+          grad(seen, s[v], dp[v], lv[v], dl[v], &pv, &dsv, &bad);
+          p[v] = pv;
+          ds[v] = dsv;
+        }
+        at_accumulate<D>(gt + row * X::P, p, dv, i, g);
+        at_accumulate<D>(qt + row * X::P, ds, dk, i, g);
+      }
+    }
+  } else {
+    // This lane's rows of a block, as (query, head of the group): the own row of the dots and the four of the sums, moved on by
+    // 4 x 16 rows without a division. Rows past the last one are read from it; their weights are 0.
+    const int step_q = 64 / a.rep, step_h = 64 - step_q * a.rep;
+    auto move = [&](AtRow& x) {
+      x.query += step_q;
+      x.head += step_h;
+      if (x.head >= a.rep) {
+        x.head -= a.rep;
+        ++x.query;
+      }
+    };
+    auto inside = [&](const AtRow& x) { return x.query < a.tq ? x : AtRow{a.tq - 1, a.rep - 1}; };
+    // A block comes straight into the first two products' operands, a block ahead (a whole one where there are registers for
+    // two); the other form goes through LDS of the wave's own.
+    constexpr int SETS = D <= 64 ? 2 : 1;
+    AtDotBlock<D, float> qn[SETS], gn[SETS];
+    float lse_n[SETS][4], delta_n[SETS][4];
+    float* const own_q = lds + rw * (2 * 16 * X::P);
+    float* const own_g = own_q + 16 * X::P;
+    int u = u0 + rw;
+    AtRow row = at_unpack(16 * u + i, a.rep), four[4];  // of the block that is fetched next
+#pragma unroll
+    for (int j = 0; j < 4; ++j) four[j] = at_unpack(16 * u + 4 * g + j, a.rep);
+    int query[4];  // of the block in hand
+    auto fetch = [&](int set) {
+      const AtRow x = inside(row);
+      qn[set].fetch(qb + x.head * a.q_h + static_cast<long>(x.query) * a.q_t, g);
+      gn[set].fetch(gb + x.head * a.o_h + static_cast<long>(x.query) * a.o_t, g);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const AtRow y = inside(four[j]);
+        const long at = (stat_b + y.head) * a.tq + y.query;
+        lse_n[set][j] = a.lse[at];
+        delta_n[set][j] = a.delta[at];
+      }
+    };
+    auto advance = [&]() {
+      move(row);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        query[j] = four[j].query;
+        move(four[j]);
+      }
+    };
+    auto step = [&](int set) {
+      __builtin_amdgcn_wave_barrier();  // the previous block has been read
+      at_stage<D>(qn[set], own_q, i, g);
+      at_stage<D>(gn[set], own_g, i, g);
+      __builtin_amdgcn_wave_barrier();
+      advance();
+      if constexpr (SETS == 2) fetch(set ^ 1);
+      const floatx4_a s = qn[set].dot(k), dp = gn[set].dot(v4);
+      float lv[4], dl[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        lv[j] = lse_n[set][j] * AT_LOG2E;
+        dl[j] = delta_n[set][j];
+      }
+      if constexpr (SETS == 1) fetch(set);
       floatx4_a p, ds;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int packed = u * AT_ROWS + row + 4 * g + v, query = at_unpack(packed, a.rep).query;
-        const bool seen = packed < rows && key < a.tk && key <= query && (a.window == 0 || query < key + a.window);
+        const bool seen = query[v] < a.tq && key < a.tk && key <= query[v] && (a.window == 0 || query[v] < key + a.window);
         float pv, dsv;
         grad(seen, s[v], dp[v], lv[v], dl[v], &pv, &dsv, &bad);
         p[v] = pv;
         ds[v] = dsv;
       }
-      at_accumulate<D>(gt + row * X::P, p, dv, i, g);
-      at_accumulate<D>(qt + row * X::P, ds, dk, i, g);
+      at_accumulate<D>(own_g, p, dv, i, g);
+      at_accumulate<D>(own_q, ds, dk, i, g);
+    };
+    if (u < u1) fetch(0);
+    for (; u < u1; u += RW * SETS) {
+      step(0);
+      if constexpr (SETS == 2) {
+        if (u + RW >= u1) break;
+        step(1);
+      }
     }
   }
   const bool split = gridDim.z > 1;
@@ -846,20 +1059,28 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_parts_kernel(Sdpa32Args a, 
   if (!(dev_finite(t.x) && dev_finite(t.y) && dev_finite(t.z) && dev_finite(t.w))) dev_raise_fault(a.fault, a.tag);
 }
 
-// Rows (keys) per workgroup: 64, or 16 with the waves splitting the other side where 64 would leave compute units
-// without a workgroup (8 x 4 heads x 256: forward 17.5 -> 12.9 us, backward 46 -> 34; 4 heads x 2048: 114 -> 69, 241 -> 190).
-bool at_narrow(omx_ctx* ctx, long planes, long rows) { return planes * ((rows + 63) / 64) < ctx->cu_count; }
+// Rows (keys) per workgroup: 64 that share every tile of the other side in LDS, or 16 whose waves take that side's blocks in
+// turn, straight into operands, with no barrier before they meet. The second is ahead where 64 would leave compute units without a
+// workgroup, and over a long other side (`span`) at any size: nothing waits for a tile there (16 heads x 4096: forward 587 ->
+// 432 us, backward 1868 -> 1446; 2 x 12 x 1024: 92 -> 67, 290 -> 222; 8 x 12 x 512: 71 -> 78, 217 -> 266); over a short one its
+// first loads and the meeting weigh more (16 x 12 x 64: 7.3 -> 8.7, 21 -> 26).
+bool at_narrow(omx_ctx* ctx, long planes, long rows, long span) {
+  const long blocks = planes * ((rows + 63) / 64), units = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  return span >= 1024 || blocks < (span >= 512 ? 2 * units : span > 128 ? units : units / 2);
+}
+// What one row's, or key's, other side comes to.
+long at_span(const Sdpa32Args& a) { return a.window > 0 ? std::min<long>(a.tk, a.window + 15l) : a.tk; }
 
 // Rows per workgroup of the forward.
-long forward_rows(omx_ctx* ctx, int dim, long planes, long rows, bool bf16_cache) {
+long forward_rows(omx_ctx* ctx, int dim, long planes, long rows, long span, bool bf16_cache) {
   if (dim >= 64 && bf16_cache)  // Twice the rows on a key's way only where half as many workgroups still fill the chip.
     return dim == 64 && (rows + 31) / 32 * planes >= 4l * (ctx->cu_count > 0 ? ctx->cu_count : 256) ? 32 : 16;
-  return at_narrow(ctx, planes, rows) ? 16 : 64;
+  return at_narrow(ctx, planes, rows, span) ? 16 : 64;
 }
 
 template <int D>
 int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) {
-  const long rows = static_cast<long>(a.tq) * a.rep, per = forward_rows(ctx, D, planes, rows, bf16_cache);
+  const long rows = static_cast<long>(a.tq) * a.rep, per = forward_rows(ctx, D, planes, rows, at_span(a), bf16_cache);
   const dim3 grid(static_cast<unsigned>((rows + per - 1) / per), planes, static_cast<unsigned>(std::max(1, a.nparts)));
   if constexpr (D >= 64) {
     if (bf16_cache) {  // (attention over a cache has no lse)
@@ -890,16 +1111,16 @@ template <int D>
 int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
   const long rows = static_cast<long>(a.tq) * a.rep;
   {
-    const bool narrow = at_narrow(ctx, planes, rows);
+    const bool narrow = at_narrow(ctx, planes, rows, at_span(a));
     const long bq = narrow ? 16 : 64;
     dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
     if (narrow) omx_launch(ctx, (sdpa32_dq_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
     else omx_launch(ctx, (sdpa32_dq_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);
     OMX_LAUNCH_CHECK(ctx, "sdpa32_dq_kernel");
   }
-  const bool narrow = at_narrow(ctx, planes, a.tk);
+  const bool narrow = at_narrow(ctx, planes, a.tk, at_span(a) * a.rep);
   const long bk = narrow ? 16 : 64, blocks = (a.tk + bk - 1) / bk;
-  // Split the rows until there are two workgroups per compute unit, as long as a share keeps two tiles (a part
+  // Split the rows until there are two workgroups per compute unit, as long as a share keeps two tiles of 64 (a part
   // costs its write, its read and a launch).
   const long seen = a.window > 0 ? std::min<long>(a.tk, a.window + bk) : a.tk;
   const long tiles = std::max<long>(1, seen * a.rep / AT_ROWS);
@@ -941,7 +1162,7 @@ bool omx_sdpa32_supports(uint64_t dim, uint64_t planes, std::initializer_list<co
 // 206 -> 30; 1024 positions 12.5 -> 11 and 28 -> 14. (The kernels for few rows: 85, 85; 82, 88; 24, 24.)
 int omx_sdpa32_key_parts(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache) {
   const long rows = static_cast<long>(a.tq) * a.rep, planes = static_cast<long>(batch) * a.kv_heads;
-  const long per = forward_rows(ctx, dim, planes, rows, bf16_cache), blocks = (rows + per - 1) / per * planes;
+  const long per = forward_rows(ctx, dim, planes, rows, at_span(a), bf16_cache), blocks = (rows + per - 1) / per * planes;
   const bool prompt = dim >= 64 && bf16_cache;
   const long keys = prompt ? 4 * (4096 / dim) : AT_ROWS;
   const double step = prompt ? (dim == 64 ? 2.0 : 1.45) : 0.5 + 0.0175 * dim;
