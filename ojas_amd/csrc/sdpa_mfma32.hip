@@ -27,10 +27,15 @@
 // its rows over the grid when keys alone do not fill the chip, and a second launch adds the parts in order.
 // No atomics; every sum has a fixed order.
 //
+// A step whose rows see every one of its keys (all but the diagonal's and a window's ends) is told by scalar compares and takes
+// no mask; rows are rescaled only where one of the wave's has a new maximum; a lane's address is 32 bits beside a scalar. With a mask
+// on every score and 64-bit addresses: forward / backward 68 / 222 us -> 64 / 198 at 2 x 12 x 1024 x 64, 26 / 103 -> 25 / 96 at 2 x 8
+// over 2 x 777, 154 / 557 -> 147 / 494 at 4 x 8 x 1024 x 128.
+//
 // On vector instructions, through shared tiles and now, us, forward / backward (batch x heads over KV heads x time x head
-// dim): 8 x 4/4 x 256 x 64: 38 / 109, 13 / 34, 11 / 32; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370, 20 / 66, 18 / 59; 16 x 12/12
-// x 512 x 64 (shared tiles still): 272 / 1337, 132 / 439 (48 and 37 TFLOP/s, causal-counted); 1 x 2/1 x 3000 x 128: 696 / 3334, 151 /
-// 409, 89 / 237.
+// dim): 8 x 4/4 x 256 x 64: 38 / 109, 13 / 34, 11 / 30; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370, 20 / 66, 19 / 60; 16 x 12/12
+// x 512 x 64 (shared tiles still): 272 / 1337, 132 / 439 (48 and 37 TFLOP/s, causal-counted); 16 x 4096 x 64: 587 / 1868 through shared
+// tiles, 382 / 1290; 1 x 2/1 x 3000 x 128: 696 / 3334, 151 / 409, 85 / 269.
 #include <algorithm>
 #include <cmath>
 
@@ -100,21 +105,31 @@ struct AtTile {
 };
 
 // ---- without LDS: a wave that shares its 16-row blocks with no other reads them straight into operands
-__device__ __forceinline__ float4 at_widen(const float4& v) { return v; }
-__device__ __forceinline__ float4 at_widen(const uint2& w) {
-  return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
-                     __uint_as_float(w.y & 0xffff0000u));
+// Rows are addressed as a scalar plus a 32-bit lane offset, so that a block whose rows lie in order needs no vector arithmetic
+// for its addresses (64-bit ones took half as many issue slots as the products). The empty assembly keeps the compiler
+// from moving the scalar part into vector registers.
+typedef const __attribute__((address_space(1))) char* AtBytes;
+__device__ __forceinline__ AtBytes at_bytes(const void* p) { return (AtBytes)(p); }
+template <typename V>
+__device__ __forceinline__ V at_load(AtBytes at, unsigned off) {
+  asm("" : "+s"(at));
+  return *reinterpret_cast<const __attribute__((address_space(1))) V*>(at + off);
+}
+template <typename T, int N>
+using AtVec = T __attribute__((ext_vector_type(N)));
+__device__ __forceinline__ float4 at_widen(const AtVec<float, 4>& v) { return make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ float4 at_widen(const AtVec<unsigned short, 4>& v) {
+  return make_float4(dev_bf16_bits_to_f32(v[0]), dev_bf16_bits_to_f32(v[1]), dev_bf16_bits_to_f32(v[2]), dev_bf16_bits_to_f32(v[3]));
 }
 __device__ __forceinline__ float at_value(float v) { return v; }
 __device__ __forceinline__ float at_value(unsigned short v) { return dev_bf16_bits_to_f32(v); }
-// One block for at_dot: lane i's row (`row` points to it), pieces 4 g of each 16 columns.
+// One block for at_dot: lane i's row, pieces 4 g of each 16 columns. `off`: bytes from `at` to the row's element 4 g.
 template <int D, typename T>
 struct AtDotBlock {
-  using Raw = std::conditional_t<sizeof(T) == 4, float4, uint2>;
-  Raw raw[AtDim<D>::S];
-  __device__ __forceinline__ void fetch(const T* row, int g) {
+  AtVec<T, 4> raw[AtDim<D>::S];
+  __device__ __forceinline__ void fetch(AtBytes at, unsigned off) {
 #pragma unroll
-    for (int s = 0; s < AtDim<D>::S; ++s) raw[s] = *reinterpret_cast<const Raw*>(row + 16 * s + 4 * g);
+    for (int s = 0; s < AtDim<D>::S; ++s) raw[s] = at_load<AtVec<T, 4>>(at + 16 * s * sizeof(T), off);
   }
   __device__ __forceinline__ floatx4_a dot(const float4 (&own)[AtDim<D>::S]) const {
     floatx4_a acc = at_zero();
@@ -133,21 +148,18 @@ struct AtDotBlock {
 template <int D>
 __device__ __forceinline__ void at_stage(const AtDotBlock<D, float>& block, float* tile16, int i, int g) {
 #pragma unroll
-  for (int s = 0; s < AtDim<D>::S; ++s) *reinterpret_cast<float4*>(tile16 + i * AtDim<D>::P + 16 * s + 4 * g) = block.raw[s];
+  for (int s = 0; s < AtDim<D>::S; ++s) *reinterpret_cast<AtVec<float, 4>*>(tile16 + i * AtDim<D>::P + 16 * s + 4 * g) = block.raw[s];
 }
-// One block for at_accumulate: rows 4 g + j (`rows[j]` point to them), columns VW i .. of each 64 (of 32, of 16).
+// One block for at_accumulate: rows 4 g + j, columns VW i .. of each 64 (of 32, of 16). `off`: bytes to row 4 g + j's element VW i.
 template <int D, typename T>
 struct AtSumBlock {
   using X = AtDim<D>;
-  T raw[4][X::NC][X::VW];
-  template <typename F>
-  __device__ __forceinline__ void fetch(F row_at, int i) {
+  AtVec<T, X::VW> raw[4][X::NC];
+  __device__ __forceinline__ void fetch(AtBytes at, const unsigned (&off)[4]) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const T* row = row_at(j) + X::VW * i;
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int c = 0; c < X::NC; ++c) __builtin_memcpy(raw[j][c], __builtin_assume_aligned(row + 64 * c, X::VW * sizeof(T)), X::VW * sizeof(T));
-    }
+      for (int c = 0; c < X::NC; ++c) raw[j][c] = at_load<AtVec<T, X::VW>>(at + 64 * c * sizeof(T), off[j]);
   }
   __device__ __forceinline__ void accumulate(const floatx4_a& weight, floatx4_a (&out)[X::S]) const {
 #pragma unroll
@@ -249,6 +261,19 @@ __device__ __forceinline__ AtRow at_unpack(int r, int rep) {
   }
   return x;
 }
+// at_unpack in a loop: a multiplication for the division (exact while r * rep < 2^32: with m = ceil(2^32 / rep), r m / 2^32 is
+// above r / rep by less than r / 2^32).
+struct AtUnpack {
+  int rep;
+  unsigned magic;
+  __device__ __forceinline__ explicit AtUnpack(int rep_) : rep(rep_), magic(rep_ == 1 ? 0u : 0xffffffffu / static_cast<unsigned>(rep_) + 1u) {}
+  __device__ __forceinline__ AtRow operator()(int r) const {
+    AtRow x;
+    x.query = rep == 1 ? r : static_cast<int>(__umulhi(static_cast<unsigned>(r), magic));
+    x.head = r - x.query * rep;
+    return x;
+  }
+};
 // Own row `r` of a [.., row, D] tensor as a product operand.
 template <int D>
 __device__ __forceinline__ void at_own(const float* row, float4 (&own)[AtDim<D>::S], int g) {
@@ -260,8 +285,8 @@ __device__ __forceinline__ void at_own(const float* row, float4 (&own)[AtDim<D>:
 template <int D, int KW, typename TK>
 __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   using X = AtDim<D>;
-  // KW = 4: nothing but the waves' sums goes through LDS, and the keys go round in blocks of 16 BLOCKS.
-  constexpr int QW = 4 / KW, BQ = 16 * QW, BLOCKS = KW == 1 ? 4 : D <= 64 ? 2 : 1, KEYS = 16 * BLOCKS;
+  // KW = 4: nothing but the waves' sums goes through LDS; a wave takes 16 keys of each 64, BLOCKS times 64 a step.
+  constexpr int QW = 4 / KW, BQ = 16 * QW, BLOCKS = KW == 1 ? 4 : D <= 64 ? 2 : 1, NEXT = KW == 1 ? 16 : 64;  // from block to block
   __shared__ __align__(16) float lds[KW == 1 ? 2 * AT_ROWS * X::P : 128 + 4 * X::S * 256];
   float* kt = lds;
   float* vt = lds + AT_ROWS * X::P;
@@ -279,7 +304,7 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   const int low = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
   const int first_pos = a.q_pos0 + at_unpack(r0, a.rep).query;
   const int last_pos = a.q_pos0 + at_unpack(min(r0 + BQ, rows) - 1, a.rep).query;
-  int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / KEYS, t_last = last_pos / KEYS;
+  int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / AT_ROWS, t_last = last_pos / AT_ROWS;
   at_key_part(a, &t_first, &t_last);
   const TK* kb = static_cast<const TK*>(a.k) + b * a.k_b + kvh * a.k_h;
   const TK* vb = static_cast<const TK*>(a.v) + b * a.k_b + kvh * a.k_h;
@@ -294,29 +319,48 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   for (int m = 0; m < X::S; ++m) o[m] = at_zero();
   float mx = -INFINITY, sum = 0.0f;  // in the exp2 domain; `sum` over this lane's keys only
   bool bad = false;
-  // Scores to weights for `key0` and the keys after it: masks, the running maximum, the rescaling that it asks for.
+  // Scores to weights for `key0` and the keys after it: masks where a row or its window ends among them, the running maximum,
+  // the rescaling that it asks for where one of the wave's rows has a new one.
+  const int end_pos = min(last_pos, t_last * AT_ROWS + AT_ROWS - 1);  // (a part of the keys ends with tile t_last)
+  const int whole_to = r0 + BQ <= rows ? min(first_pos, end_pos) : -1, whole_from = a.window > 0 ? max(0, last_pos + 1 - a.window) : 0;
+  const int high = min(pos, end_pos);
+  float check = 0.0f;  // NaN once a score that counts was not finite
   auto weights = [&](floatx4_a (&s)[BLOCKS], int key0) {
     float top = -INFINITY;
+    if (key0 + (BLOCKS - 1) * NEXT + 15 <= whole_to && key0 >= whole_from) {  // (uniform)
 #pragma unroll
-    for (int n = 0; n < BLOCKS; ++n)
+      for (int n = 0; n < BLOCKS; ++n)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int key = key0 + n * 16 + 4 * g + v;
-        const bool seen = key <= pos && key >= low;
-        const float x = s[n][v] * scale2;
-        bad |= seen && !dev_finite(x);
-        s[n][v] = seen ? x : -INFINITY;
-        top = fmaxf(top, s[n][v]);
-      }
+        for (int v = 0; v < 4; ++v) {
+          s[n][v] *= scale2;
+          check = fmaf(s[n][v], 0.0f, check);
+          top = fmaxf(top, s[n][v]);
+        }
+    } else {
+#pragma unroll
+      for (int n = 0; n < BLOCKS; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int key = key0 + n * NEXT + 4 * g + v;
+          const bool seen = key <= high && key >= low;
+          const float x = s[n][v] * scale2;
+          bad |= seen && !dev_finite(x);
+          s[n][v] = seen ? x : -INFINITY;
+          top = fmaxf(top, s[n][v]);
+        }
+    }
     top = at_row_max(top);
-    const float mx_new = fmaxf(mx, top), base = mx_new == -INFINITY ? 0.0f : mx_new;
-    const float rescale = __builtin_amdgcn_exp2f(mx - base);  // 0 on the first keys; 1 when none were seen yet: the sums are 0
-    mx = mx_new;
-    sum *= rescale;
+    if (__any(top > mx)) {
+      const float mx_new = fmaxf(mx, top);
+      const float rescale = mx_new == mx ? 1.0f : __builtin_amdgcn_exp2f(mx - mx_new);  // 0 on the first keys
+      mx = mx_new;
+      sum *= rescale;
 #pragma unroll
-    for (int m = 0; m < X::S; ++m)
+      for (int m = 0; m < X::S; ++m)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) o[m][v] *= rescale;
+        for (int v = 0; v < 4; ++v) o[m][v] *= rescale;
+    }
+    const float base = mx == -INFINITY ? 0.0f : mx;
 #pragma unroll
     for (int n = 0; n < BLOCKS; ++n)
 #pragma unroll
@@ -345,7 +389,7 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
       floatx4_a s[BLOCKS];
 #pragma unroll
       for (int n = 0; n < BLOCKS; ++n) s[n] = at_dot<D>(kt + n * 16 * X::P, q, i, g);
-      weights(s, t * KEYS);
+      weights(s, t * AT_ROWS);
 #pragma unroll
       for (int n = 0; n < BLOCKS; ++n) at_accumulate<D>(vt + n * 16 * X::P, s[n], o, i, g);
     }
@@ -354,25 +398,57 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
     // the last one are read from it; their weights are 0.)
     AtDotBlock<D, TK> keys[BLOCKS];
     AtSumBlock<D, TK> values[BLOCKS];
+    // Up to `straight` the keys lie in order and whole (beyond: the ring's end, or the last key).
+    const int straight = min(a.tk, a.capacity - a.slot0);
+    const unsigned pitch = static_cast<unsigned>(a.k_t) * sizeof(TK);
+    unsigned k_off = i * pitch + 4 * g * sizeof(TK), v_off[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v_off[j] = (4 * g + j) * pitch + X::VW * i * sizeof(TK);
+    // A block's first row, and row `r` of it from there.
+    auto block_at = [&](const TK* base, int key0) { return at_bytes(base + (key0 + 16 <= straight ? (a.slot0 + key0) * a.k_t : 0l)); };
+    auto row_off = [&](int key0, int r) {
+      const unsigned int slot = static_cast<unsigned int>(a.slot0) + min(key0 + r, a.tk - 1), capacity = a.capacity;
+      return (slot >= capacity ? slot - capacity : slot) * pitch;
+    };
+    // This wave's block of tile `t`, and whether a row of the workgroup sees any of it.
+    const int from_pos = a.window > 0 ? max(0, first_pos + 1 - a.window) : 0;
+    auto block_of = [&](int t) { return t * AT_ROWS + kw * 16; };
+    auto counts = [&](int key0) { return key0 <= end_pos && key0 + 15 >= from_pos; };
     auto fetch = [&](int t) {
 #pragma unroll
-      for (int n = 0; n < BLOCKS; ++n) keys[n].fetch(kb + slot_at(min(t * KEYS + n * 16 + i, a.tk - 1)), g);
+      for (int n = 0; n < BLOCKS; ++n) {
+        const int key0 = min(block_of(t + n), end_pos & ~15);  // (one that does not count reads the last that does)
+        unsigned off = k_off;
+        if (key0 + 16 > straight) off = row_off(key0, i) + 4 * g * sizeof(TK);
+        keys[n].fetch(block_at(kb, key0), off);
+      }
     };
-    int t = t_first + kw;
-    if (t <= t_last) fetch(t);
-    for (; t <= t_last; t += KW) {
+    if (t_first <= t_last) fetch(t_first);
+    for (int t = t_first; t <= t_last; t += BLOCKS) {
 #pragma unroll
-      for (int n = 0; n < BLOCKS; ++n)
-        values[n].fetch([&](int j) { return vb + slot_at(min(t * KEYS + n * 16 + 4 * g + j, a.tk - 1)); }, i);
+      for (int n = 0; n < BLOCKS; ++n) {
+        const int key0 = min(block_of(t + n), end_pos & ~15);
+        unsigned off[4] = {v_off[0], v_off[1], v_off[2], v_off[3]};
+        if (key0 + 16 > straight) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) off[j] = row_off(key0, 4 * g + j) + X::VW * i * sizeof(TK);
+        }
+        values[n].fetch(block_at(vb, key0), off);
+      }
       floatx4_a s[BLOCKS];
 #pragma unroll
-      for (int n = 0; n < BLOCKS; ++n) s[n] = keys[n].dot(q);
-      fetch(min(t + KW, t_last));
-      weights(s, t * KEYS);
+      for (int n = 0; n < BLOCKS; ++n) {
+        s[n] = at_zero();
+        if (counts(block_of(t + n))) s[n] = keys[n].dot(q);
+      }
+      fetch(min(t + BLOCKS, t_last));
+      weights(s, block_of(t));
 #pragma unroll
-      for (int n = 0; n < BLOCKS; ++n) values[n].accumulate(s[n], o);
+      for (int n = 0; n < BLOCKS; ++n)
+        if (counts(block_of(t + n))) values[n].accumulate(s[n], o);
     }
   }
+  bad |= check != 0.0f;
   sum = at_row_sum(sum);
   float* out = a.out + b * a.o_b + (static_cast<long>(kvh) * a.rep + at.head) * a.o_h + static_cast<long>(at.query) * a.o_t;
   float* lse = a.lse ? a.lse + (static_cast<long>(b) * a.kv_heads * a.rep + static_cast<long>(kvh) * a.rep + at.head) * a.tq + at.query : nullptr;
@@ -709,6 +785,13 @@ struct AtGrad {
     *p = pr;
     *ds = seen ? scale * (pr * (dp - delta)) : 0.0f;
   }
+  // The same for a score that is seen; `check` turns NaN where the other form says bad.
+  __device__ __forceinline__ void whole(float score, float dp, float lse2, float delta, float* p, float* ds, float* check) const {
+    const float x = score * scale2;
+    *p = __builtin_amdgcn_exp2f(x - lse2);
+    *check = fmaf(x, 0.0f, fmaf(*p, 0.0f, *check));
+    *ds = scale * (*p * (dp - delta));
+  }
 };
 
 // dQ, and the row term delta = dO . O when `out` is given (it is read from `delta` otherwise).
@@ -759,14 +842,18 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
 #pragma unroll
   for (int m = 0; m < X::S; ++m) dq[m] = at_zero();
   bool bad = false;
-  // dS of keys key0 + 4 g + v, from the scores and dP.
+  // dS of keys key0 + 4 g + v, from the scores and dP; without masks where every row sees them all.
+  const int whole_to = r0 + BQ <= rows ? first_pos : -1, whole_from = a.window > 0 ? max(0, last_pos + 1 - a.window) : 0;
+  float check = 0.0f;
   auto slopes = [&](const floatx4_a& s, const floatx4_a& dp, int key0) {
     floatx4_a ds;
+    const bool whole = key0 + 15 <= whole_to && key0 >= whole_from;  // (uniform)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int key = key0 + 4 * g + v;
       float p, d;
-      grad(key <= pos && key >= low, s[v], dp[v], lse2, delta, &p, &d, &bad);
+      if (whole) grad.whole(s[v], dp[v], lse2, delta, &p, &d, &check);
+      else grad(key <= pos && key >= low, s[v], dp[v], lse2, delta, &p, &d, &bad);
       ds[v] = d;
     }
     return ds;
@@ -797,10 +884,13 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
     // LDS of the wave's own. (Keys past the last one are read from it; their dS is 0.)
     AtDotBlock<D, float> keys[2], values[2];
     float* const own = lds + kw * (16 * X::P);
+    const unsigned pitch = static_cast<unsigned>(a.k_t) * 4u, off0 = i * pitch + 16u * g;
     auto fetch = [&](int set, int t) {
-      const long at_key = static_cast<long>(min(t * KEYS + i, a.tk - 1)) * a.k_t;
-      keys[set].fetch(kb + at_key, g);
-      values[set].fetch(vb + at_key, g);
+      const int key0 = t * KEYS;
+      unsigned off = off0;
+      if (key0 + KEYS > a.tk) off = min(i, a.tk - 1 - key0) * pitch + 16u * g;
+      keys[set].fetch(at_bytes(kb + key0 * a.k_t), off);
+      values[set].fetch(at_bytes(vb + key0 * a.k_t), off);
     };
     auto step = [&](int set, int t) {
       __builtin_amdgcn_wave_barrier();  // the previous block has been read
@@ -818,6 +908,7 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
       step(1, t + KW);
     }
   }
+  bad |= check != 0.0f;
   float* out = a.gq + q_at;
   if constexpr (KW == 1) {
     if (r < rows) bad |= at_store<D, 4>(out, dq, 1.0f, g, 0);
@@ -926,18 +1017,10 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
       }
     }
   } else {
-    // This lane's rows of a block, as (query, head of the group): the own row of the dots and the four of the sums, moved on by
-    // 4 x 16 rows without a division. Rows past the last one are read from it; their weights are 0.
-    const int step_q = 64 / a.rep, step_h = 64 - step_q * a.rep;
-    auto move = [&](AtRow& x) {
-      x.query += step_q;
-      x.head += step_h;
-      if (x.head >= a.rep) {
-        x.head -= a.rep;
-        ++x.query;
-      }
-    };
-    auto inside = [&](const AtRow& x) { return x.query < a.tq ? x : AtRow{a.tq - 1, a.rep - 1}; };
+    // Rows past the last one are read from it; their weights are 0.
+    const AtUnpack unpack(a.rep);
+    const unsigned q_pitch = static_cast<unsigned>(a.q_t) * 4u, o_pitch = static_cast<unsigned>(a.o_t) * 4u;
+    const unsigned q_head = static_cast<unsigned>(a.q_h) * 4u, o_head = static_cast<unsigned>(a.o_h) * 4u;
     // A block comes straight into the first two products' operands, a block ahead (a whole one where there are registers for
     // two); the other form goes through LDS of the wave's own.
     constexpr int SETS = D <= 64 ? 2 : 1;
@@ -946,37 +1029,46 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
     float* const own_q = lds + rw * (2 * 16 * X::P);
     float* const own_g = own_q + 16 * X::P;
     int u = u0 + rw;
-    AtRow row = at_unpack(16 * u + i, a.rep), four[4];  // of the block that is fetched next
+    float check = 0.0f;
+    // Where 16 rows are whole queries of the group (1, 2, 4, 8 or 16 heads) a block's offsets from its first row never change.
+    const bool even = 16 % a.rep == 0;
+    const AtRow own0 = unpack(i);
+    const unsigned q_off0 = own0.head * q_head + own0.query * q_pitch + 16u * g, g_off0 = own0.head * o_head + own0.query * o_pitch + 16u * g;
+    unsigned stat0[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) four[j] = at_unpack(16 * u + 4 * g + j, a.rep);
-    int query[4];  // of the block in hand
-    auto fetch = [&](int set) {
-      const AtRow x = inside(row);
-      qn[set].fetch(qb + x.head * a.q_h + static_cast<long>(x.query) * a.q_t, g);
-      gn[set].fetch(gb + x.head * a.o_h + static_cast<long>(x.query) * a.o_t, g);
+    for (int j = 0; j < 4; ++j) {
+      const AtRow y = unpack(4 * g + j);
+      stat0[j] = (static_cast<unsigned>(y.head) * a.tq + y.query) * 4u;
+    }
+    auto fetch = [&](int set, int u_next) {
+      const int first = 16 * u_next;
+      const bool in_order = even && first + 16 <= rows;
+      const long query0 = in_order ? unpack(first).query : 0;
+      unsigned q_off = q_off0, g_off = g_off0, stat[4] = {stat0[0], stat0[1], stat0[2], stat0[3]};
+      if (!in_order) {
+        const AtRow x = unpack(min(first + i, rows - 1));
+        q_off = x.head * q_head + x.query * q_pitch + 16u * g;
+        g_off = x.head * o_head + x.query * o_pitch + 16u * g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const AtRow y = unpack(min(first + 4 * g + j, rows - 1));
+          stat[j] = (static_cast<unsigned>(y.head) * a.tq + y.query) * 4u;
+        }
+      }
+      qn[set].fetch(at_bytes(qb + query0 * a.q_t), q_off);
+      gn[set].fetch(at_bytes(gb + query0 * a.o_t), g_off);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const AtRow y = inside(four[j]);
-        const long at = (stat_b + y.head) * a.tq + y.query;
-        lse_n[set][j] = a.lse[at];
-        delta_n[set][j] = a.delta[at];
+        lse_n[set][j] = at_load<float>(at_bytes(a.lse + stat_b * a.tq + query0), stat[j]);
+        delta_n[set][j] = at_load<float>(at_bytes(a.delta + stat_b * a.tq + query0), stat[j]);
       }
     };
-    auto advance = [&]() {
-      move(row);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        query[j] = four[j].query;
-        move(four[j]);
-      }
-    };
-    auto step = [&](int set) {
+    auto step = [&](int set, int u_now) {
       __builtin_amdgcn_wave_barrier();  // the previous block has been read
       at_stage<D>(qn[set], own_q, i, g);
       at_stage<D>(gn[set], own_g, i, g);
       __builtin_amdgcn_wave_barrier();
-      advance();
-      if constexpr (SETS == 2) fetch(set ^ 1);
+      if constexpr (SETS == 2) fetch(set ^ 1, min(u_now + RW, u1 - 1));
       const floatx4_a s = qn[set].dot(k), dp = gn[set].dot(v4);
       float lv[4], dl[4];
 #pragma unroll
@@ -984,27 +1076,36 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
         lv[j] = lse_n[set][j] * AT_LOG2E;
         dl[j] = delta_n[set][j];
       }
-      if constexpr (SETS == 1) fetch(set);
+      if constexpr (SETS == 1) fetch(set, min(u_now + RW, u1 - 1));
+      // Without masks where the block's first and last queries see every key (uniform).
+      const int from = unpack(16 * u_now).query, to = unpack(16 * u_now + 15).query;
+      const bool whole = from >= j0 + BK - 1 && 16 * u_now + 16 <= rows && j0 + BK <= a.tk && (a.window == 0 || to < j0 + a.window);
       floatx4_a p, ds;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const bool seen = query[v] < a.tq && key < a.tk && key <= query[v] && (a.window == 0 || query[v] < key + a.window);
         float pv, dsv;
-        grad(seen, s[v], dp[v], lv[v], dl[v], &pv, &dsv, &bad);
+        if (whole) {
+          grad.whole(s[v], dp[v], lv[v], dl[v], &pv, &dsv, &check);
+        } else {
+          const int packed = 16 * u_now + 4 * g + v, query = unpack(packed).query;
+          const bool seen = packed < rows && key < a.tk && key <= query && (a.window == 0 || query < key + a.window);
+          grad(seen, s[v], dp[v], lv[v], dl[v], &pv, &dsv, &bad);
+        }
         p[v] = pv;
         ds[v] = dsv;
       }
       at_accumulate<D>(own_g, p, dv, i, g);
       at_accumulate<D>(own_q, ds, dk, i, g);
     };
-    if (u < u1) fetch(0);
+    if (u < u1) fetch(0, u);
     for (; u < u1; u += RW * SETS) {
-      step(0);
+      step(0, u);
       if constexpr (SETS == 2) {
         if (u + RW >= u1) break;
-        step(1);
+        step(1, u + RW);
       }
     }
+    bad |= check != 0.0f;
   }
   const bool split = gridDim.z > 1;
   const long plane = static_cast<long>(a.tk) * D;  // parts: [z][b, kv head][tk][D], dK's then dV's
@@ -1062,9 +1163,14 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_parts_kernel(Sdpa32Args a, 
 // Rows (keys) per workgroup: 64 that share every tile of the other side in LDS, or 16 whose waves take that side's blocks in
 // turn, straight into operands, with no barrier before they meet. The second is ahead where 64 would leave compute units without a
 // workgroup, and over a long other side (`span`) at any size: nothing waits for a tile there (16 heads x 4096: forward 587 ->
-// 432 us, backward 1868 -> 1446; 2 x 12 x 1024: 92 -> 67, 290 -> 222; 8 x 12 x 512: 71 -> 78, 217 -> 266); over a short one its
+// 382 us, backward 1868 -> 1290; 2 x 12 x 1024: 92 -> 64, 290 -> 198; 8 x 12 x 512: 71 -> 78, 217 -> 266); over a short one its
 // first loads and the meeting weigh more (16 x 12 x 64: 7.3 -> 8.7, 21 -> 26).
-bool at_narrow(omx_ctx* ctx, long planes, long rows, long span) {
+bool at_narrow(omx_ctx* ctx, const Sdpa32Args& a, long planes, long rows, long span) {
+  // The second form's lane offsets are 32 bits of bytes over a plane, its row numbers 32 bits times the group's heads.
+  const long limit = 1l << 30, heads = a.rep - 1l;
+  if (a.capacity * a.k_t >= limit || a.tk * a.k_t >= limit || a.tq * a.q_t + heads * a.q_h >= limit || a.tq * a.o_t + heads * a.o_h >= limit ||
+      (static_cast<long>(a.tq) * a.rep + 64) * a.rep >= 4 * limit)
+    return false;
   const long blocks = planes * ((rows + 63) / 64), units = ctx->cu_count > 0 ? ctx->cu_count : 256;
   return span >= 1024 || blocks < (span >= 512 ? 2 * units : span > 128 ? units : units / 2);
 }
@@ -1072,15 +1178,15 @@ bool at_narrow(omx_ctx* ctx, long planes, long rows, long span) {
 long at_span(const Sdpa32Args& a) { return a.window > 0 ? std::min<long>(a.tk, a.window + 15l) : a.tk; }
 
 // Rows per workgroup of the forward.
-long forward_rows(omx_ctx* ctx, int dim, long planes, long rows, long span, bool bf16_cache) {
+long forward_rows(omx_ctx* ctx, const Sdpa32Args& a, int dim, long planes, long rows, bool bf16_cache) {
   if (dim >= 64 && bf16_cache)  // Twice the rows on a key's way only where half as many workgroups still fill the chip.
     return dim == 64 && (rows + 31) / 32 * planes >= 4l * (ctx->cu_count > 0 ? ctx->cu_count : 256) ? 32 : 16;
-  return at_narrow(ctx, planes, rows, span) ? 16 : 64;
+  return at_narrow(ctx, a, planes, rows, at_span(a)) ? 16 : 64;
 }
 
 template <int D>
 int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) {
-  const long rows = static_cast<long>(a.tq) * a.rep, per = forward_rows(ctx, D, planes, rows, at_span(a), bf16_cache);
+  const long rows = static_cast<long>(a.tq) * a.rep, per = forward_rows(ctx, a, D, planes, rows, bf16_cache);
   const dim3 grid(static_cast<unsigned>((rows + per - 1) / per), planes, static_cast<unsigned>(std::max(1, a.nparts)));
   if constexpr (D >= 64) {
     if (bf16_cache) {  // (attention over a cache has no lse)
@@ -1111,14 +1217,14 @@ template <int D>
 int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
   const long rows = static_cast<long>(a.tq) * a.rep;
   {
-    const bool narrow = at_narrow(ctx, planes, rows, at_span(a));
+    const bool narrow = at_narrow(ctx, a, planes, rows, at_span(a));
     const long bq = narrow ? 16 : 64;
     dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
     if (narrow) omx_launch(ctx, (sdpa32_dq_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
     else omx_launch(ctx, (sdpa32_dq_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);
     OMX_LAUNCH_CHECK(ctx, "sdpa32_dq_kernel");
   }
-  const bool narrow = at_narrow(ctx, planes, a.tk, at_span(a) * a.rep);
+  const bool narrow = at_narrow(ctx, a, planes, a.tk, at_span(a) * a.rep);
   const long bk = narrow ? 16 : 64, blocks = (a.tk + bk - 1) / bk;
   // Split the rows until there are two workgroups per compute unit, as long as a share keeps two tiles of 64 (a part
   // costs its write, its read and a launch).
@@ -1162,7 +1268,7 @@ bool omx_sdpa32_supports(uint64_t dim, uint64_t planes, std::initializer_list<co
 // 206 -> 30; 1024 positions 12.5 -> 11 and 28 -> 14. (The kernels for few rows: 85, 85; 82, 88; 24, 24.)
 int omx_sdpa32_key_parts(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache) {
   const long rows = static_cast<long>(a.tq) * a.rep, planes = static_cast<long>(batch) * a.kv_heads;
-  const long per = forward_rows(ctx, dim, planes, rows, at_span(a), bf16_cache), blocks = (rows + per - 1) / per * planes;
+  const long per = forward_rows(ctx, a, dim, planes, rows, bf16_cache), blocks = (rows + per - 1) / per * planes;
   const bool prompt = dim >= 64 && bf16_cache;
   const long keys = prompt ? 4 * (4096 / dim) : AT_ROWS;
   const double step = prompt ? (dim == 64 ? 2.0 : 1.45) : 0.5 + 0.0175 * dim;
