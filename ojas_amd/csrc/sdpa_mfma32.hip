@@ -30,12 +30,13 @@
 // A step whose rows see every one of its keys (all but the diagonal's and a window's ends) is told by scalar compares and takes
 // no mask; rows are rescaled only where one of the wave's has a new maximum; a lane's address is 32 bits beside a scalar. With a mask
 // on every score and 64-bit addresses: forward / backward 68 / 222 us -> 64 / 198 at 2 x 12 x 1024 x 64, 26 / 103 -> 25 / 96 at 2 x 8
-// over 2 x 777, 154 / 557 -> 147 / 494 at 4 x 8 x 1024 x 128.
+// over 2 x 777, 154 / 557 -> 147 / 494 at 4 x 8 x 1024 x 128. With a plane's blocks on few L2s (at_place) from there: 48 / 154,
+// 23 / 88, 107 / 366.
 //
 // On vector instructions, through shared tiles and now, us, forward / backward (batch x heads over KV heads x time x head
 // dim): 8 x 4/4 x 256 x 64: 38 / 109, 13 / 34, 11 / 30; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370, 20 / 66, 19 / 60; 16 x 12/12
 // x 512 x 64 (shared tiles still): 272 / 1337, 132 / 439 (48 and 37 TFLOP/s, causal-counted); 16 x 4096 x 64: 587 / 1868 through shared
-// tiles, 382 / 1290; 1 x 2/1 x 3000 x 128: 696 / 3334, 151 / 409, 85 / 269.
+// tiles, 325 / 1120; 1 x 2/1 x 3000 x 128: 696 / 3334, 151 / 409, 85 / 269.
 #include <algorithm>
 #include <cmath>
 
@@ -233,6 +234,18 @@ __device__ __forceinline__ bool at_store(float* row, const floatx4_a (&out)[AtDi
   return bad;
 }
 
+// This workgroup's block of rows (or keys) and its (batch, KV head) plane. Workgroups go round-robin over the 8 XCDs by their linear
+// index, and each XCD has its own L2: planes are dealt so that one is read through as few of them as their number allows (one
+// where it is a multiple of 8, all eight where it is odd), its blocks in turn over those. With a plane's blocks over all eight, 12
+// heads x 64 of 4 sequences, 256 new positions of 700: 72 MB came from beyond the L2s for 9 of keys and values.
+struct AtPlace {
+  int block, plane;
+};
+__device__ __forceinline__ AtPlace at_place() {
+  const unsigned planes = gridDim.y, share = min(8u, planes & (0u - planes));
+  const unsigned index = blockIdx.y * gridDim.x + blockIdx.x, n = index / share, run = n / gridDim.x;
+  return {static_cast<int>(n - run * gridDim.x), static_cast<int>(index % share + share * run)};
+}
 // Where part blockIdx.z of a row's result goes (Sdpa32Args::partial).
 __device__ __forceinline__ float* at_partial(const Sdpa32Args& a, int dim, int b, int kvh, int query, int head) {
   const long row = (static_cast<long>(b) * a.tq + query) * a.kv_heads * a.rep + static_cast<long>(kvh) * a.rep + head;
@@ -292,9 +305,10 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
   float* vt = lds + AT_ROWS * X::P;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int qw = wave % QW, kw = wave / QW;
-  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const AtPlace place = at_place();
+  const int b = place.plane / a.kv_heads, kvh = place.plane - b * a.kv_heads;
   const int rows = a.tq * a.rep;
-  const int r0 = (gridDim.x - 1 - blockIdx.x) * BQ;  // the rows that see the most keys first
+  const int r0 = (gridDim.x - 1 - place.block) * BQ;  // the rows that see the most keys first
   const int r = r0 + qw * 16 + i;
   const AtRow at = at_unpack(min(r, rows - 1), a.rep);
   const long q_at = b * a.q_b + (static_cast<long>(kvh) * a.rep + at.head) * a.q_h + static_cast<long>(at.query) * a.q_t;
@@ -523,10 +537,12 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_fwd_kernel(Sdpa32Args a) {
 // A workgroup takes 16 MB rows and its four waves share the keys, AtPrompt::KEYS at a time. No wave reads another's
 // keys, so keys go from memory straight into fragments and only values pass through LDS, a region per wave, where
 // the transposing reads form the other operand: no barrier before the waves meet. The next keys and values are on
-// their way during softmax and the second product. Bound by vector instructions: softmax and the cuts.
-// us on f32 instructions -> here (relative error against 64 bits): 4 x 12 heads x 64, 256 new positions of 700: 38.6 -> 20.6
-// (2.5e-7 -> 1.5e-7); 8 x 16 over 4 KV heads x 64, 512 of 1024: 173 -> 85 (5.2e-7 -> 1.6e-7); 2 x 8 over 2 x 128, 100 of 800:
-// 41 -> 16 (2.9e-7 -> 1.7e-7).
+// their way during softmax and the second product. A step that every row sees whole takes no mask, rows are rescaled only where a
+// maximum moves, addresses are a scalar and 32 bits (half of the vector instructions went there). Bound by the way from the L2s
+// (13 TB/s of keys and values; without the loads three quarters of the time) and by vector instructions: softmax and the cuts.
+// us on f32 instructions, on bf16 ones, with neither masks nor planes over all L2s (relative error against 64 bits): 4 x 12 heads x
+// 64, 256 new positions of 700: 38.6, 20.5, 17.5 (2.5e-7, 1.5e-7, the same); 8 x 16 over 4 KV heads x 64, 512 of 1024: 173, 85, 67
+// (5.2e-7, 1.6e-7); 2 x 8 over 2 x 128, 100 of 800: 41, 16, 13.7 (2.9e-7, 1.5e-7); 16 x 12 x 64, 256 of 1000: 77, 58 from there.
 typedef __bf16 bf16x8_a __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4_a __attribute__((ext_vector_type(4)));
 typedef short short4_a __attribute__((ext_vector_type(4)));
@@ -547,12 +563,9 @@ struct AtParts {
     }
   }
 };
-// acc += A . (the parts), A's lane values 8 g + j beside theirs.
-__device__ __forceinline__ floatx4_a at_mfma_parts(u32x4_a a, const AtParts& b, floatx4_a acc) {
-#pragma unroll
-  for (int n = 2; n >= 0; --n)
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_a, a), __builtin_bit_cast(bf16x8_a, b.part[n]), acc, 0, 0, 0);
-  return acc;
+// acc += A . B, lane values 8 g + j of both. A sum takes an operand's parts smallest first.
+__device__ __forceinline__ floatx4_a at_mfma16(u32x4_a a, u32x4_a b, floatx4_a acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_a, a), __builtin_bit_cast(bf16x8_a, b), acc, 0, 0, 0);
 }
 
 template <int D>
@@ -570,10 +583,11 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
   using X = AtPrompt<D>;
   __shared__ __align__(16) char lds[4 * X::KEYS * X::PITCH];
   static_assert(512 + 4 * X::DB * 1024 <= 4 * X::KEYS * X::PITCH, "the waves' sums fit");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
-  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
+  const AtPlace place = at_place();
+  const int b = place.plane / a.kv_heads, kvh = place.plane - b * a.kv_heads;
   const int rows = a.tq * a.rep;
-  const int r0 = (gridDim.x - 1 - blockIdx.x) * (16 * MB);  // the rows that see the most keys first
+  const int r0 = (gridDim.x - 1 - place.block) * (16 * MB);  // the rows that see the most keys first
   AtRow at[MB];
   AtParts q[MB][X::KS];
   int pos[MB], low[MB];
@@ -595,32 +609,46 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
   const int last_pos = a.q_pos0 + at_unpack(min(r0 + 16 * MB, rows) - 1, a.rep).query;
   int t_first = (a.window > 0 ? max(0, first_pos + 1 - a.window) : 0) / X::KEYS, t_last = last_pos / X::KEYS;
   if constexpr (SPLIT) at_key_part(a, &t_first, &t_last);
+  const int last_low = a.window > 0 ? max(0, last_pos + 1 - a.window) : 0;
   const unsigned short* kb = static_cast<const unsigned short*>(a.k) + b * a.k_b + kvh * a.k_h;
   const unsigned short* vb = static_cast<const unsigned short*>(a.v) + b * a.k_b + kvh * a.k_h;
   char* region = lds + wave * (X::KEYS * X::PITCH);
 
   u32x4_a kn[X::NB][X::KS], vn[X::PIECES];
-  auto slot_at = [&](int key) {
-    // A ring wraps at most once over the keys that are read (slot0 + key can pass 2^31).
-    const unsigned int slot = static_cast<unsigned int>(a.slot0) + key, capacity = a.capacity;
-    return static_cast<long>(slot >= capacity ? slot - capacity : slot) * a.k_t;
-  };
-  auto fetch = [&](int t) {  // keys past the last one are rows of zeros
+  // Rows by 32-bit lane offsets from the tile's first row, or, past the ring's end, from the ring's first (at_prompt). Keys past
+  // the last one are read from it; their weights are 0.
+  const int straight = min(a.tk, a.capacity - a.slot0);  // up to here the keys lie in order
+  const unsigned pitch = 2u * static_cast<unsigned>(a.k_t);
+  const unsigned k_off = i * pitch + 16 * g, v_off = lane / (D / 8) * pitch + lane % (D / 8) * 16;
+  auto fetch = [&](int t) {
+    const int key0 = t * X::KEYS;
+    const bool plain = key0 + X::KEYS <= straight;                          // (uniform)
+    const unsigned row0 = plain || straight == a.tk ? a.slot0 + key0 : 0u;  // the first row
+    unsigned k_at[X::NB], v_at[X::PIECES];
+    if (plain) {
+      unsigned step = pitch;
+      asm("" : "+s"(step));  // (twelve sums rather than twelve registers across the loop)
 #pragma unroll
-    for (int n = 0; n < X::NB; ++n) {
-      const int key = t * X::KEYS + n * 16 + i;
+      for (int n = 0; n < X::NB; ++n) k_at[n] = k_off + n * 16 * step;
 #pragma unroll
-      for (int s = 0; s < X::KS; ++s) {
-        if (key < a.tk) kn[n][s] = *reinterpret_cast<const u32x4_a*>(kb + slot_at(key) + 32 * s + 8 * g);
-        else kn[n][s] = u32x4_a{0u, 0u, 0u, 0u};
-      }
+      for (int p = 0; p < X::PIECES; ++p) v_at[p] = v_off + p * (512 / D) * step;
+    } else {
+      auto row_off = [&](int row) {
+        const unsigned slot = static_cast<unsigned>(a.slot0) + min(key0 + row, a.tk - 1), capacity = a.capacity;
+        return ((slot >= capacity ? slot - capacity : slot) - row0) * pitch;
+      };
+#pragma unroll
+      for (int n = 0; n < X::NB; ++n) k_at[n] = row_off(n * 16 + i) + 16 * g;
+#pragma unroll
+      for (int p = 0; p < X::PIECES; ++p) v_at[p] = row_off(lane / (D / 8) + p * (512 / D)) + lane % (D / 8) * 16;
     }
+    const AtBytes ka = at_bytes(kb + row0 * a.k_t), va = at_bytes(vb + row0 * a.k_t);
 #pragma unroll
-    for (int p = 0; p < X::PIECES; ++p) {
-      const int idx = lane + 64 * p, key = t * X::KEYS + idx / (D / 8);
-      if (key < a.tk) vn[p] = *reinterpret_cast<const u32x4_a*>(vb + slot_at(key) + idx % (D / 8) * 8);
-      else vn[p] = u32x4_a{0u, 0u, 0u, 0u};
-    }
+    for (int n = 0; n < X::NB; ++n)
+#pragma unroll
+      for (int s = 0; s < X::KS; ++s) kn[n][s] = at_load<u32x4_a>(ka + 64 * s, k_at[n]);
+#pragma unroll
+    for (int p = 0; p < X::PIECES; ++p) vn[p] = at_load<u32x4_a>(va, v_at[p]);
   };
 
   const float scale2 = a.scale * AT_LOG2E;
@@ -633,6 +661,7 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
 #pragma unroll
     for (int d = 0; d < X::DB; ++d) o[m][d] = at_zero();
   }
+  float least = 0.0f;  // of the scores that no mask looked at: minus infinity where one is; NaN and infinity show in the sums
   bool bad = false;
   if (t_first + wave <= t_last) fetch(t_first + wave);
   for (int t = t_first + wave; t <= t_last; t += 4) {
@@ -652,32 +681,49 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
       for (int m = 0; m < MB; ++m) {
         s[m][n] = at_zero();
 #pragma unroll
-        for (int ks = 0; ks < X::KS; ++ks) s[m][n] = at_mfma_parts(kn[n][ks], q[m][ks], s[m][n]);
+        for (int ks = 0; ks < X::KS; ++ks)
+#pragma unroll
+          for (int part = 2; part >= 0; --part) s[m][n] = at_mfma16(kn[n][ks], q[m][ks].part[part], s[m][n]);
       }
     if (t + 4 <= t_last) fetch(t + 4);
+    const bool whole = t * X::KEYS + X::KEYS - 1 <= first_pos && t * X::KEYS >= last_low;  // (uniform)
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
       float top = -INFINITY;
+      if (whole) {
 #pragma unroll
-      for (int n = 0; n < X::NB; ++n)
+        for (int n = 0; n < X::NB; ++n)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int key = t * X::KEYS + n * 16 + 4 * g + v;
-          const bool seen = key <= pos[m] && key >= low[m];
-          const float x = s[m][n][v] * scale2;
-          bad |= seen && !dev_finite(x);
-          s[m][n][v] = seen ? x : -INFINITY;
-          top = fmaxf(top, s[m][n][v]);
-        }
+          for (int v = 0; v < 4; ++v) {
+            s[m][n][v] *= scale2;
+            top = fmaxf(top, s[m][n][v]);
+            least = fminf(least, s[m][n][v]);
+          }
+      } else {
+#pragma unroll
+        for (int n = 0; n < X::NB; ++n)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int key = t * X::KEYS + n * 16 + 4 * g + v;
+            const bool seen = key <= pos[m] && key >= low[m];
+            const float x = s[m][n][v] * scale2;
+            bad |= seen && !dev_finite(x);
+            s[m][n][v] = seen ? x : -INFINITY;
+            top = fmaxf(top, s[m][n][v]);
+          }
+      }
       top = at_row_max(top);
-      const float mx_new = fmaxf(mx[m], top), base = mx_new == -INFINITY ? 0.0f : mx_new;
-      const float rescale = __builtin_amdgcn_exp2f(mx[m] - base);
-      mx[m] = mx_new;
-      sum[m] *= rescale;
+      if (__any(top > mx[m])) {
+        const float mx_new = fmaxf(mx[m], top);
+        const float rescale = mx_new == mx[m] ? 1.0f : __builtin_amdgcn_exp2f(mx[m] - mx_new);  // 0 on the first keys
+        mx[m] = mx_new;
+        sum[m] *= rescale;
 #pragma unroll
-      for (int d = 0; d < X::DB; ++d)
+        for (int d = 0; d < X::DB; ++d)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) o[m][d][v] *= rescale;
+          for (int v = 0; v < 4; ++v) o[m][d][v] *= rescale;
+      }
+      const float base = mx[m] == -INFINITY ? 0.0f : mx[m];
 #pragma unroll
       for (int n = 0; n < X::NB; ++n)
 #pragma unroll
@@ -696,6 +742,7 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
                             s[m][2 * h + 1][0], s[m][2 * h + 1][1], s[m][2 * h + 1][2], s[m][2 * h + 1][3]};
         p[m].cut(x);
       }
+      u32x4_a value[X::DB];
 #pragma unroll
       for (int d = 0; d < X::DB; ++d) {
         typedef short4_a __attribute__((address_space(3))) * lds_ptr;
@@ -703,12 +750,20 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && MB == 1 ? 3 : 2) void sdpa_p
         const short4_a lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at_v));
         const short4_a hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at_v + 16 * X::PITCH));
         const uint2 l = __builtin_bit_cast(uint2, lo), u = __builtin_bit_cast(uint2, hi);
-        const u32x4_a value = {l.x, l.y, u.x, u.y};
-#pragma unroll
-        for (int m = 0; m < MB; ++m) o[m][d] = at_mfma_parts(value, p[m], o[m][d]);
+        value[d] = u32x4_a{l.x, l.y, u.x, u.y};
       }
+#pragma unroll
+      for (int n = 2; n >= 0; --n)  // over all sums between two products of one: these wait for each other (17.8 -> 17.5 us at 4 x 12, 256 of 700)
+#pragma unroll
+        for (int d = 0; d < X::DB; ++d)
+#pragma unroll
+          for (int m = 0; m < MB; ++m)
+            o[m][d] = at_mfma16(value[d], p[m].part[n], o[m][d]);
     }
   }
+  bad |= least == -INFINITY;
+#pragma unroll
+  for (int m = 0; m < MB; ++m) bad |= !dev_finite(sum[m]);
   // The four waves' shares of the same rows: wave w adds up the column blocks w, w + 4, ...
   float* stat = reinterpret_cast<float*>(lds);                // [4][2][16]
   float4* part = reinterpret_cast<float4*>(lds + 512);        // [4][DB][64]
@@ -805,9 +860,10 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
   float* vt = lds + AT_ROWS * X::P;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int qw = wave % QW, kw = wave / QW;
-  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const AtPlace place = at_place();
+  const int b = place.plane / a.kv_heads, kvh = place.plane - b * a.kv_heads;
   const int rows = a.tq * a.rep;
-  const int r0 = (gridDim.x - 1 - blockIdx.x) * BQ;
+  const int r0 = (gridDim.x - 1 - place.block) * BQ;
   const int r = r0 + qw * 16 + i;
   const AtRow at = at_unpack(min(r, rows - 1), a.rep);
   const long head = static_cast<long>(kvh) * a.rep + at.head;
@@ -945,9 +1001,10 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
   float* delta_t = lse_t + AT_ROWS;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int kg = wave % KG, rw = wave / KG;
-  const int b = blockIdx.y / a.kv_heads, kvh = blockIdx.y - b * a.kv_heads;
+  const AtPlace place = at_place();
+  const int b = place.plane / a.kv_heads, kvh = place.plane - b * a.kv_heads;
   const int rows = a.tq * a.rep;
-  const int j0 = blockIdx.x * BK, key = j0 + kg * 16 + i;
+  const int j0 = place.block * BK, key = j0 + kg * 16 + i;
   const long k_at = b * a.k_b + kvh * a.k_h + static_cast<long>(min(key, a.tk - 1)) * a.k_t;
   float4 k[X::S], v4[X::S];
   at_own<D>(static_cast<const float*>(a.k) + k_at, k, g);
@@ -1109,7 +1166,7 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
   }
   const bool split = gridDim.z > 1;
   const long plane = static_cast<long>(a.tk) * D;  // parts: [z][b, kv head][tk][D], dK's then dV's
-  const long part_at = ((static_cast<long>(blockIdx.z) * gridDim.y + blockIdx.y) * a.tk + min(key, a.tk - 1)) * D;
+  const long part_at = ((static_cast<long>(blockIdx.z) * gridDim.y + place.plane) * a.tk + min(key, a.tk - 1)) * D;
   float* ok = split ? a.parts + part_at : a.gk + k_at;
   float* ov = split ? a.parts + static_cast<long>(gridDim.z) * gridDim.y * plane + part_at : a.gv + k_at;
   if constexpr (RW == 1) {
@@ -1163,7 +1220,7 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_parts_kernel(Sdpa32Args a, 
 // Rows (keys) per workgroup: 64 that share every tile of the other side in LDS, or 16 whose waves take that side's blocks in
 // turn, straight into operands, with no barrier before they meet. The second is ahead where 64 would leave compute units without a
 // workgroup, and over a long other side (`span`) at any size: nothing waits for a tile there (16 heads x 4096: forward 587 ->
-// 382 us, backward 1868 -> 1290; 2 x 12 x 1024: 92 -> 64, 290 -> 198; 8 x 12 x 512: 71 -> 78, 217 -> 266); over a short one its
+// 382 us, backward 1868 -> 1290; 2 x 12 x 1024: 92 -> 64, 290 -> 198; 8 x 12 x 512: 71 -> 78, 217 -> 266; planes over all L2s); over a short one its
 // first loads and the meeting weigh more (16 x 12 x 64: 7.3 -> 8.7, 21 -> 26).
 bool at_narrow(omx_ctx* ctx, const Sdpa32Args& a, long planes, long rows, long span) {
   // The second form's lane offsets are 32 bits of bytes over a plane, its row numbers 32 bits times the group's heads.
@@ -1177,9 +1234,16 @@ bool at_narrow(omx_ctx* ctx, const Sdpa32Args& a, long planes, long rows, long s
 // What one row's, or key's, other side comes to.
 long at_span(const Sdpa32Args& a) { return a.window > 0 ? std::min<long>(a.tk, a.window + 15l) : a.tk; }
 
+// sdpa_prompt_kernel: bf16 caches of wider heads, unless a ring's rows lie past 32 bits of lane offset from its first (4 GiB and
+// more of one batch entry's keys) and the keys that are read run past its end.
+bool at_prompt(const Sdpa32Args& a, int dim, bool bf16_cache) {
+  const bool wraps = static_cast<long>(a.slot0) + a.tk > a.capacity;
+  return dim >= 64 && bf16_cache && a.k_t < 1l << 24 && !(wraps && a.capacity * a.k_t >= 1l << 31);
+}
+
 // Rows per workgroup of the forward.
 long forward_rows(omx_ctx* ctx, const Sdpa32Args& a, int dim, long planes, long rows, bool bf16_cache) {
-  if (dim >= 64 && bf16_cache)  // Twice the rows on a key's way only where half as many workgroups still fill the chip.
+  if (at_prompt(a, dim, bf16_cache))  // Twice the rows on a key's way only where half as many workgroups still fill the chip.
     return dim == 64 && (rows + 31) / 32 * planes >= 4l * (ctx->cu_count > 0 ? ctx->cu_count : 256) ? 32 : 16;
   return at_narrow(ctx, a, planes, rows, at_span(a)) ? 16 : 64;
 }
@@ -1189,7 +1253,7 @@ int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) 
   const long rows = static_cast<long>(a.tq) * a.rep, per = forward_rows(ctx, a, D, planes, rows, bf16_cache);
   const dim3 grid(static_cast<unsigned>((rows + per - 1) / per), planes, static_cast<unsigned>(std::max(1, a.nparts)));
   if constexpr (D >= 64) {
-    if (bf16_cache) {  // (attention over a cache has no lse)
+    if (at_prompt(a, D, bf16_cache)) {  // (attention over a cache has no lse)
       const bool two = per == 32, split = a.nparts > 1;  // (two: four workgroups per compute unit and more, never split)
       if constexpr (D == 64) {
         if (two) omx_launch(ctx, (sdpa_prompt_kernel<D, 2, false>), grid, dim3(AT_THREADS), 0, a);
@@ -1200,13 +1264,12 @@ int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) 
     }
   }
   const bool narrow = per == 16;
-  using Cache = std::conditional_t<(D < 64), unsigned short, float>;  // bf16 caches of wider heads are gone by now
-  auto launch_bf16 = [&](auto kernel) { omx_launch(ctx, kernel, grid, dim3(AT_THREADS), 0, a); };
+  using Cache = std::conditional_t<(D < 64), unsigned short, float>;  // bf16 caches of wider heads: prompt or (past 32 bits) wide
   if (narrow) {
-    if (bf16_cache) launch_bf16(&sdpa32_fwd_kernel<D, 4, Cache>);
+    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, Cache>), grid, dim3(AT_THREADS), 0, a);
     else omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, float>), grid, dim3(AT_THREADS), 0, a);
   } else {
-    if (bf16_cache) launch_bf16(&sdpa32_fwd_kernel<D, 1, Cache>);
+    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, unsigned short>), grid, dim3(AT_THREADS), 0, a);
     else omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, float>), grid, dim3(AT_THREADS), 0, a);
   }
   OMX_LAUNCH_CHECK(ctx, "sdpa32_fwd_kernel");
@@ -1269,7 +1332,7 @@ bool omx_sdpa32_supports(uint64_t dim, uint64_t planes, std::initializer_list<co
 int omx_sdpa32_key_parts(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, bool bf16_cache) {
   const long rows = static_cast<long>(a.tq) * a.rep, planes = static_cast<long>(batch) * a.kv_heads;
   const long per = forward_rows(ctx, a, dim, planes, rows, bf16_cache), blocks = (rows + per - 1) / per * planes;
-  const bool prompt = dim >= 64 && bf16_cache;
+  const bool prompt = at_prompt(a, dim, bf16_cache);
   const long keys = prompt ? 4 * (4096 / dim) : AT_ROWS;
   const double step = prompt ? (dim == 64 ? 2.0 : 1.45) : 0.5 + 0.0175 * dim;
   const long steps = (a.tk + keys - 1) / keys, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;

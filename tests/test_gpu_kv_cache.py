@@ -256,6 +256,36 @@ def test_prompt_chunks_over_bf16_caches_lose_nothing(be, b, tq, h, hkv, d, capac
 
 
 @pytest.mark.parametrize("b,tq,h,hkv,d,capacity,kv_len,window", [
+    (1, 17, 2, 2, 64, 320, 320, None), (1, 64, 4, 2, 64, 300, 700, 200), (1, 40, 2, 2, 128, 150, 411, 110), (1, 33, 3, 3, 64, 200, 197, 130),
+    (32, 40, 16, 16, 64, 257, 250, None), (1, 24, 2, 1, 128, 129, 129, 97)])
+def test_prompt_tiles_that_every_row_sees(be, b, tq, h, hkv, d, capacity, kv_len, window):
+    """Tiles of 64 keys (32 of head dim 128) without masks: whole ones, the ring's end in one, the last key in one, a window
+    that starts in one. Bound as above. What such a tile holds that is not finite raises: a key whose score overflows, to
+    either side, a value that is not a number."""
+    print("prompt tiles", b, tq, h, hkv, d, capacity, kv_len, window, flush=True)
+    r = np.random.default_rng(tq * 5 + d)
+    q = r.standard_normal((b, tq, h, d)).astype(np.float32)
+    q[..., 0] = 10.0
+    seq = [orc.round_bf16(r.standard_normal((b, kv_len, hkv, d)).astype(np.float32)) for _ in range(2)]
+    k, v = (ring(x, capacity, kv_len, 0.0) for x in seq)
+    wide = [np.repeat(x.astype(np.float64), h // hkv, axis=2).transpose(0, 2, 1, 3) for x in seq]
+    s = q.astype(np.float64).transpose(0, 2, 1, 3) @ wide[0].transpose(0, 1, 3, 2) / np.sqrt(d)
+    at, key = kv_len - tq + np.arange(tq)[:, None], np.arange(kv_len)[None, :]
+    s = np.where((key <= at) & (key > at - (window or kv_len)), s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = ((p / p.sum(-1, keepdims=True)) @ wide[1]).transpose(0, 2, 1, 3)
+    run = lambda k, v: be.cached_attention_forward(be.upload(q), be.upload(k, BF16), be.upload(v, BF16), kv_len, window)
+    assert np.linalg.norm(be.download(run(k, v)) - want) <= 1e-6 * np.linalg.norm(want)
+    slot = (kv_len - tq - 1) % capacity  # every row sees it
+    for which, value in ((0, 3e38), (0, -3e38), (1, np.nan)):
+        broken = [k.copy(), v.copy()]
+        broken[which][-1, slot, -1, 0] = value
+        run(*broken)
+        with pytest.raises(OjasError):
+            be.sync()
+
+
+@pytest.mark.parametrize("b,tq,h,hkv,d,capacity,kv_len,window", [
     (1, 1, 16, 1, 64, 8192, 8192, None), (1, 16, 12, 12, 64, 4100, 4097, None), (1, 1, 64, 2, 128, 2048, 5000, 2048),
     (2, 70, 2, 1, 64, 3000, 2999, 700), (1, 17, 2, 2, 32, 2500, 2500, None), (1, 16, 1, 1, 16, 4000, 9000, 1500),
     (1, 33, 1, 1, 128, 1500, 1500, 1)])

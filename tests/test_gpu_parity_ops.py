@@ -1063,3 +1063,43 @@ def test_f32_attention_on_the_matrix_units(be, b, h, hkv, t, d, window):
     assert np.abs(be.download(lse) - want_lse).max() <= 1e-5 * max(1.0, float(np.abs(want_lse).max()))
     for got, ref in zip(be.causal_sdpa_backward(dq, dk, dv, out, lse, dg, window), grads):
         assert np.abs(be.download(got) - ref).max() <= 1e-5 * max(1.0, float(np.abs(ref).max()))
+
+
+@pytest.mark.parametrize("b,h,hkv,t,d,window", [(1, 2, 2, 16, 64, None), (1, 3, 1, 63, 64, None), (2, 2, 2, 64, 32, 16), (1, 4, 2, 129, 128, 64),
+                                                (1, 2, 1, 257, 64, 65), (1, 16, 1, 80, 16, None), (4, 12, 12, 192, 64, None)])
+def test_f32_attention_steps_that_every_row_sees(be, b, h, hkv, t, d, window):
+    """Steps without masks beside those that the diagonal, a window's start or the last row cuts, against 64-bit sums: t + d
+    roundings of a row's sum are under (t + d) 2^-24 of its norm if all went one way, in each of at most two sums behind a result.
+    What a step without masks holds that is not finite raises, forward and backward."""
+    from ojas_amd.backend import NON_FINITE, OjasError
+
+    print("f32 attention steps", b, h, hkv, t, d, window, flush=True)
+    r = np.random.default_rng(t + d)
+    q, gy = (r.standard_normal((b, h, t, d)).astype(np.float32) for _ in range(2))
+    k, v = (r.standard_normal((b, hkv, t, d)).astype(np.float32) for _ in range(2))
+    rep, w = h // hkv, window or t
+    q64, g64 = q.astype(np.float64), gy.astype(np.float64)
+    k64, v64 = (np.repeat(x.astype(np.float64), rep, axis=1) for x in (k, v))
+    i, j = np.arange(t)[:, None], np.arange(t)[None, :]
+    s = np.where((j <= i) & (j > i - w), q64 @ k64.transpose(0, 1, 3, 2) / np.sqrt(d), -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    want = p @ v64
+    ds = p * (g64 @ v64.transpose(0, 1, 3, 2) - (g64 * want).sum(-1, keepdims=True)) / np.sqrt(d)
+    fold = lambda x: x.reshape(b, hkv, rep, t, d).sum(2)
+    grads = (ds @ k64, fold(ds.transpose(0, 1, 3, 2) @ q64), fold(p.transpose(0, 1, 3, 2) @ g64))
+    dq, dk, dv, dg = (be.upload(x) for x in (q, k, v, gy))
+    out, lse = be.causal_sdpa_forward(dq, dk, dv, window)
+    for got, ref in zip((out,) + tuple(be.causal_sdpa_backward(dq, dk, dv, out, lse, dg, window)), (want,) + grads):
+        assert np.linalg.norm(be.download(got) - ref) <= 2.0 * (rep * t + d) * 2.0**-24 * np.linalg.norm(ref)
+    q[..., 0] = 10.0
+    at = max(0, t - min(w, 40))  # the last rows see it; where t allows, in a step of its own
+    for value in (3e38, -3e38):
+        k2 = k.copy()
+        k2[-1, -1, at, 0] = value
+        args = (be.upload(q), be.upload(k2), dv)
+        for run in (lambda: be.causal_sdpa_forward(*args, window), lambda: be.causal_sdpa_backward(*args, out, lse, dg, window)):
+            run()
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.code == NON_FINITE
