@@ -47,15 +47,24 @@ __device__ __forceinline__ void store_pack(T* __restrict__ p, size_t pack, const
   }
 }
 
+// Packs per thread: one up to four blocks per compute unit, two up to eight, BK_PACKS beyond. A few thousand rows were 16 to 176
+// blocks whose threads took their packs one latency after the other (rope over 1024 x 4 x 64 6.3 us on 32 blocks, 3.2 on 128).
+__host__ __device__ inline uint64_t packs_per_thread(uint64_t packs, uint64_t blocks) {
+  return packs <= blocks * BK_THREADS ? 1 : packs <= blocks * (2 * BK_THREADS) ? 2 : BK_PACKS;
+}
 inline dim3 pack_grid(uint64_t packs) {
-  uint64_t per_block = static_cast<uint64_t>(BK_THREADS) * BK_PACKS;
-  uint64_t blocks = (packs + per_block - 1) / per_block;
+  const uint64_t each = packs_per_thread(packs, 1024), per_block = each * BK_THREADS;
+  const uint64_t blocks = (packs + per_block - 1) / per_block;
   return dim3(static_cast<unsigned>(blocks > 0 ? blocks : 1));
 }
-#define PACK_LOOP(p, packs)                                                                          \
-  for (size_t p = static_cast<size_t>(blockIdx.x) * (BK_THREADS * BK_PACKS) + threadIdx.x,           \
-              end_ = min(static_cast<size_t>(packs), (static_cast<size_t>(blockIdx.x) + 1) * (BK_THREADS * BK_PACKS)); \
+#define PACK_LOOP(p, packs)                                                                                             \
+  for (size_t span_ = packs_per_thread(packs, gridDim.x) * BK_THREADS, p = blockIdx.x * span_ + threadIdx.x,            \
+              end_ = min(static_cast<size_t>(packs), (blockIdx.x + 1) * span_);                                          \
        p < end_; p += BK_THREADS)
+// n / d in 32 bits where they allow it (a 64-bit division is some 100 instructions).
+__device__ __forceinline__ size_t quotient(size_t n, size_t d) {
+  return ((n | d) >> 32) == 0 ? static_cast<unsigned>(n) / static_cast<unsigned>(d) : n / d;
+}
 
 // Whether every pointer allows 4-element packs of `esz`-byte elements.
 inline bool packs_of_four(uint64_t n, size_t esz, std::initializer_list<const void*> ptrs) {
@@ -168,9 +177,13 @@ __global__ __launch_bounds__(BK_THREADS) void rope_kernel(const T* __restrict__ 
   const size_t packs = rows * half_packs;
   bool bad = false;
   PACK_LOOP(p, packs) {
-    size_t row = p / half_packs;
-    int c = static_cast<int>(p % half_packs);
-    size_t trow = heads ? (row / heads) % time : row;
+    size_t row = quotient(p, half_packs);
+    int c = static_cast<int>(p - row * half_packs);
+    size_t trow = row;
+    if (heads) {
+      trow = quotient(row, heads);
+      trow -= quotient(trow, time) * time;
+    }
     float a[V], b[V], c1[V], s1[V], c2[V], s2[V], lo[V], hi[V];
     load_pack<T, V>(x, row * row_packs + c, a);
     load_pack<T, V>(x, row * row_packs + half_packs + c, b);
@@ -202,7 +215,7 @@ __global__ __launch_bounds__(BK_THREADS) void gate_sigmoid_kernel(float* __restr
                                                                   unsigned long long tag) {
   bool bad = false;
   PACK_LOOP(i, n) {
-    float u = z[i] + bias[i % heads];
+    float u = z[i] + bias[i - quotient(i, heads) * heads];
     bad |= !dev_finite(u);
     float s, rest;
     sigmoid_pair(u, &s, &rest);
@@ -220,7 +233,7 @@ __global__ __launch_bounds__(BK_THREADS) void gate_apply_kernel(const TA* __rest
   PACK_LOOP(p, packs) {
     float a[V], r[V];
     load_pack<TA, V>(attn, p, a);
-    float g = gates[p / head_packs];
+    float g = gates[quotient(p, head_packs)];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       r[j] = a[j] * g;
@@ -658,7 +671,8 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
     return omx_fail(ctx, OMX_DTYPE, "%s: attn and grad_output must share a dtype", op);
 
   // Workspace: [gates f32][gz in the operand dtype][per-block bias partials][two-stage sum scratch].
-  const int block_rows = 16;
+  // 16 rows per block, or 4 where those are under a block per compute unit (1024 rows of 4 x 64: 6.7 us on 64 blocks, 4.3 on 256).
+  const int block_rows = rows < 16ull * 256 ? 4 : 16;
   const uint64_t blocks = (rows + block_rows - 1) / block_rows;
   const uint64_t items = rows * heads;
   const uint64_t gates_bytes = round_up(items * sizeof(float), 256);

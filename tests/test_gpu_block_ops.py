@@ -596,3 +596,40 @@ def test_qkv_prepare_equals_norm_then_rope_then_blend(be, heads, kv_heads, dim, 
     close(got_gv, want_gv, BF16_TOL, "gv")
     close(be.download(gqw), want_gqw, BF16_TOL, "q norm weight gradient")
     close(be.download(gkw), want_gkw, BF16_TOL, "k norm weight gradient")
+
+
+@pytest.mark.parametrize("packs", [1, 256, 1024 * 256, 1024 * 256 + 1, 2 * 1024 * 256, 2 * 1024 * 256 + 1, 3 * 1024 * 256 + 77])
+def test_packs_per_thread_at_their_edges(be, packs):
+    """One, two or four packs of four values per thread: the last pack of the last block, and one more."""
+    n = 4 * packs
+    r = np.random.default_rng(packs)
+    a, b, gy = (r.standard_normal(n).astype(np.float32) for _ in range(3))
+    da, db, dg = (be.upload(x) for x in (a, b, gy))
+    assert np.array_equal(be.download(be.mul_forward(da, db)), a * b)
+    ga, gb = be.mul_backward(da, db, dg)
+    assert np.array_equal(be.download(ga), gy * b) and np.array_equal(be.download(gb), gy * a)
+    lam = np.zeros(1, np.float32)
+    gv, gv0, gl = be.value_residual_blend_backward(da, db, be.upload(lam), dg)
+    assert np.array_equal(be.download(gv), gy * np.float32(0.5)) and np.array_equal(be.download(gv0), gy * np.float32(0.5))
+    terms = (b.astype(np.float64) - a) * gy
+    # A thread's 16 terms, a block's tree and at most 16 blocks in turn: under 64 roundings of the terms' size.
+    assert abs(float(be.download(gl)[0]) - 0.25 * terms.sum()) <= 0.25 * 64 * 2.0**-24 * np.abs(terms).sum()
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 4097, 8191, 8193])
+@pytest.mark.parametrize("dim", [1, 63, 64, 128])
+def test_norm_backward_of_short_rows(be, rows, dim):
+    """Four rows of a wave at once, 16 or 32 of a block: every remainder, against 64-bit sums."""
+    print(f"short rows {rows}x{dim}", flush=True)
+    r = np.random.default_rng(rows * 131 + dim)
+    x, gy = (r.standard_normal((rows, dim)).astype(np.float32) + np.float32(2.0) for _ in range(2))
+    w = r.standard_normal(dim).astype(np.float32)
+    x64, g64 = x.astype(np.float64), gy.astype(np.float64)
+    rstd = 1.0 / np.sqrt((x64 * x64).mean(-1, keepdims=True) + 1e-6)
+    hat, gw = x64 * rstd, g64 * w
+    want = (gw - hat * (gw * hat).mean(-1, keepdims=True)) * rstd
+    gx, gwt = be.rms_norm_backward(be.upload(x), be.upload(w), be.upload(gy), 1e-6)
+    # 16 roundings of the two terms whose difference it is; a column's sum: at most 64 additions in turn on any path.
+    size = (np.abs(gw) + np.abs(hat) * np.abs(gw * hat).mean(-1, keepdims=True)) * rstd
+    assert (np.abs(be.download(gx) - want) <= 16 * 2.0**-24 * size).all()
+    assert (np.abs(be.download(gwt) - (g64 * hat).sum(0)) <= 64 * 2.0**-24 * np.abs(g64 * hat).sum(0)).all()
