@@ -44,17 +44,6 @@ struct KvArgs {
   unsigned long long tag;
 };
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
-}
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
 // Copies tile rows [pos0, pos0 + 64) of one KV head of both caches into LDS, widened to f32; rows
 // at or past kv_len become zeros. A lane's 16-byte pieces are chunk indices lane, lane + 64, ...
 // of the tile's 64 * dim / 4; (key0, piece0) locates chunk `lane`. Loads are issued eight keys'
@@ -247,26 +236,27 @@ constexpr int KG_ROWS = 4;  // query rows per block
 template <typename T>
 constexpr int KG_FEW_WAVES = sizeof(T) == 2 ? 16 : 8;
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
 // Sum over the LPK adjacent lanes that hold one key; every one of them receives the total.
 template <int LPK>
 __device__ __forceinline__ float group_sum(float v) {
-  if constexpr (LPK >= 2) v = dpp_add<0xB1>(v);   // quad_perm [1,0,3,2]
-  if constexpr (LPK >= 4) v = dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
-  if constexpr (LPK >= 8) v = dpp_add<0x141>(v);  // row_half_mirror
-  if constexpr (LPK >= 16) v = dpp_add<0x140>(v); // row_mirror
-  if constexpr (LPK >= 32) v += __shfl_xor(v, 16);
-  if constexpr (LPK >= 64) v += __shfl_xor(v, 32);
+  const auto add = [](float x, float y) { return x + y; };
+  if constexpr (LPK >= 2) v += dev_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+  if constexpr (LPK >= 4) v += dev_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  if constexpr (LPK >= 8) v += dev_dpp<0x141>(v);  // row_half_mirror
+  if constexpr (LPK >= 16) v += dev_dpp<0x140>(v); // row_mirror
+  if constexpr (LPK >= 32) v = dev_meet_16(v, add);
+  if constexpr (LPK >= 64) v = dev_meet_32(v, add);
   return v;
 }
 // Combines the 64 / LPK lane groups (lanes that differ in the bits at and above LPK).
 template <int LPK, typename F>
 __device__ __forceinline__ float across_groups(float v, F f) {
-#pragma unroll
-  for (int o = LPK; o < 64; o <<= 1) v = f(v, __shfl_xor(v, o));
+  if constexpr (LPK <= 1) v = f(v, dev_dpp<0xB1>(v));
+  if constexpr (LPK <= 2) v = f(v, dev_dpp<0x4E>(v));
+  if constexpr (LPK <= 4) v = f(v, __shfl_xor(v, 4));
+  if constexpr (LPK <= 8) v = f(v, dev_dpp<0x128>(v));  // row_ror 8
+  if constexpr (LPK <= 16) v = dev_meet_16(v, f);
+  if constexpr (LPK <= 32) v = dev_meet_32(v, f);
   return v;
 }
 

@@ -52,8 +52,13 @@ __device__ __forceinline__ void load8f(const float* __restrict__ p, float (&v)[8
 // Sum over the LPR adjacent lanes that hold one row.
 template <int LPR>
 __device__ __forceinline__ float row_sum(float v) {
-#pragma unroll
-  for (int m = 1; m < LPR; m <<= 1) v += __shfl_xor(v, m, 64);
+  const auto add = [](float x, float y) { return x + y; };
+  if constexpr (LPR > 1) v += dev_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+  if constexpr (LPR > 2) v += dev_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  if constexpr (LPR > 4) v += dev_dpp<0x141>(v);  // row_half_mirror: the other four lanes of eight, which agree
+  if constexpr (LPR > 8) v += dev_dpp<0x140>(v);  // row_mirror
+  if constexpr (LPR > 16) v = dev_meet_16(v, add);
+  if constexpr (LPR > 32) v = dev_meet_32(v, add);
   return v;
 }
 // sigmoid(u) and 1 - sigmoid(u), both without cancellation.
@@ -229,9 +234,7 @@ __global__ __launch_bounds__(QP_THREADS) void qkv_prepare_bwd_kernel(
   for (int which = 0; which < 2; ++which)
 #pragma unroll
     for (int i = 0; i < 8; ++i) red[which][sub][col + i] = acc_w[which][i];
-  float lam = acc_lambda;
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) lam += __shfl_xor(lam, m, 64);
+  const float lam = wave_sum(acc_lambda);
   if ((threadIdx.x & 63) == 0) red_lambda[threadIdx.x >> 6] = lam;
   __syncthreads();
   for (int i = threadIdx.x; i < 2 * D; i += QP_THREADS) {

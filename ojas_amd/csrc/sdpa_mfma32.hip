@@ -53,13 +53,9 @@ __device__ __forceinline__ floatx4_a at_mfma(float a, float b, floatx4_a c) {
 }
 __device__ __forceinline__ floatx4_a at_zero() { return floatx4_a{0.0f, 0.0f, 0.0f, 0.0f}; }
 // Over the four lanes that hold one row.
-// (v_permlane16_swap and v_permlane32_swap of a value with its copy leave both lanes' values in both: no LDS round trip)
 template <typename F>
 __device__ __forceinline__ float at_row(float v, F f) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  return dev_meet_32(dev_meet_16(v, f), f);
 }
 __device__ __forceinline__ float at_row_max(float v) { return at_row(v, [](float x, float y) { return fmaxf(x, y); }); }
 __device__ __forceinline__ float at_row_sum(float v) { return at_row(v, [](float x, float y) { return x + y; }); }
