@@ -100,6 +100,61 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(GemmArgs g) {
   if (bad) dev_raise_fault(g.fault, g.tag);
 }
 
+// The same for up to four rows and few columns: four columns per workgroup, so that four times as many compute units read the
+// weights. The 16 row and the 16 column places of a product are 4 rows or columns x 4 quarters of K; of its 256 sums the 64 whose two
+// quarters agree are kept (lanes l16 / 4 == lane / 16), and a workgroup's 4 columns x K come in loads as wide as before. One row, 768
+// columns, us in a decode step:
+// K = 768 3.7 -> 3.0, K = 3072 6.2 -> 3.9 (16 columns there were 12 steps a wave, four at a time, and 98 KB a compute unit).
+template <int WAVES, int CHUNK, bool PLAIN>
+__global__ __launch_bounds__(WAVES * 64) void gemm_rows4_kernel(GemmArgs g) {
+  __shared__ float red[WAVES * 64];  // [wave][quarter][row][column]
+  gemm_select_batch(g, blockIdx.z);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, quarter = l16 >> 2, col0 = blockIdx.x * 4;
+  const long k0 = static_cast<long>(quarter) * (g.K / 4) + (lane >> 4) * 8;
+  // Rows and columns past the end are read from the last one and never stored.
+  const unsigned short* a = static_cast<const unsigned short*>(g.a) + static_cast<long>(min(l16 & 3, g.M - 1)) * g.lda + k0;
+  const unsigned short* b = static_cast<const unsigned short*>(g.b) + static_cast<long>(min(col0 + (l16 & 3), g.N - 1)) * g.ldb + k0;
+  floatx4_s acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  const int steps = g.K / 128;
+  const int s_end = steps * (wave + 1) / WAVES;
+  for (int s0 = steps * wave / WAVES; s0 < s_end; s0 += CHUNK) {
+    const int live = min(CHUNK, s_end - s0);  // uniform over the wave
+    u32x4_s bf[CHUNK], af[CHUNK];
+#pragma unroll
+    for (int s = 0; s < CHUNK; ++s)
+      if (s < live) {
+        bf[s] = *reinterpret_cast<const u32x4_s*>(b + (s0 + s) * 32);
+        af[s] = *reinterpret_cast<const u32x4_s*>(a + (s0 + s) * 32);
+      }
+#pragma unroll
+    for (int s = 0; s < CHUNK; ++s)
+      if (s < live)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_s, bf[s]), __builtin_bit_cast(bf16x8_s, af[s]), acc, 0, 0, 0);
+  }
+  // acc[v]: row place l16, column place 4 * (lane / 16) + v.
+  if (quarter == lane >> 4) *reinterpret_cast<floatx4_s*>(red + wave * 64 + l16 * 4) = acc;
+  __syncthreads();
+  if (wave != 0) return;
+  // Lane: row lane / 16, quarter lane / 4 % 4, column lane % 4. Neighbours first, then the quarters.
+  float part[WAVES];
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) part[w] = red[w * 64 + (quarter * 4 + (lane >> 4)) * 4 + (lane & 3)];
+#pragma unroll
+  for (int span = 1; span < WAVES; span *= 2)
+#pragma unroll
+    for (int w = 0; w < WAVES; w += 2 * span) part[w] += part[w + span];
+  float x = part[0];
+  x += dev_dpp<0x128>(x);  // row_ror 8, 4: the quarter two away, then the other two
+  x += dev_dpp<0x124>(x);
+  const float x0 = dev_dpp<0x00>(x), x1 = dev_dpp<0x55>(x), x2 = dev_dpp<0xAA>(x), x3 = dev_dpp<0xFF>(x);  // quad_perm: one column to all
+  const int row = lane >> 4;
+  if (l16 == 0 && row < g.M) {
+    const bool bad = PLAIN ? gemm_store4(g, 0, row, col0, x0, x1, x2, x3) : gemm_store4_epi(g, 0, row, col0, x0, x1, x2, x3);
+    if (bad) dev_raise_fault(g.fault, g.tag);
+  }
+}
+
 struct SkinnyTile {
   int mb, nb;
 };
@@ -131,8 +186,7 @@ int skinny_tile(const GemmArgs& g, long units) {
 template <int MB, int NB, int WAVES>
 int32_t launch_skinny_waves(omx_ctx* ctx, const GemmArgs& g) {
   constexpr int smem = WAVES * MB * NB * 1024;
-  auto kernel = g.epi == OMX_EPI_NONE ? &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK, true>
-                                      : &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK, false>;
+  auto kernel = g.epi == OMX_EPI_NONE ? &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK, true> : &gemm_skinny_kernel<MB, NB, WAVES, SKINNY_CHUNK, false>;
   if constexpr (smem > 64 * 1024)
     OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
   dim3 grid(static_cast<unsigned>((g.N + 16 * NB - 1) / (16 * NB)), static_cast<unsigned>((g.M + 16 * MB - 1) / (16 * MB)),
@@ -141,10 +195,23 @@ int32_t launch_skinny_waves(omx_ctx* ctx, const GemmArgs& g) {
   OMX_LAUNCH_CHECK(ctx, "gemm_skinny_kernel");
   return OMX_OK;
 }
-// Eight waves share K; up to 512 columns four do (two to four steps each), with half the sums to meet.
+// Eight waves share K; up to 512 columns four do (two to four steps each), with half the sums to meet. (Sixteen over K = 3072, six
+// steps in flight each: 64 rows by 768 columns 8.4 -> 8.9 us.)
 template <int MB, int NB>
 int32_t launch_skinny(omx_ctx* ctx, const GemmArgs& g) {
   return g.K <= 512 ? launch_skinny_waves<MB, NB, 4>(ctx, g) : launch_skinny_waves<MB, NB, 8>(ctx, g);
+}
+
+// Four rows at most, a workgroup per four columns at most one per compute unit, quarters of K whole steps.
+bool rows4(const GemmArgs& g, long units) { return g.M <= 4 && g.K % 128 == 0 && (g.N + 3l) / 4 * g.batches <= units; }
+int32_t launch_rows4(omx_ctx* ctx, const GemmArgs& g) {
+  const bool plain = g.epi == OMX_EPI_NONE, few = g.K <= 1024;
+  auto kernel = few ? (plain ? &gemm_rows4_kernel<4, 2, true> : &gemm_rows4_kernel<4, 2, false>)
+                    : (plain ? &gemm_rows4_kernel<8, 4, true> : &gemm_rows4_kernel<8, 4, false>);
+  dim3 grid(static_cast<unsigned>((g.N + 3) / 4), 1, static_cast<unsigned>(g.batches));
+  omx_launch_timed(ctx, kernel, grid, dim3(few ? 256 : 512), 0, ctx->timing_start, ctx->timing_stop, g);
+  OMX_LAUNCH_CHECK(ctx, "gemm_rows4_kernel");
+  return OMX_OK;
 }
 
 }  // namespace
@@ -158,6 +225,7 @@ double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km,
 }
 
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g) {
+  if (rows4(g, ctx->cu_count > 0 ? ctx->cu_count : 256)) return launch_rows4(ctx, g);
   switch (skinny_tile(g, ctx->cu_count > 0 ? ctx->cu_count : 256)) {
     case 0: return launch_skinny<1, 1>(ctx, g);
     case 1: return launch_skinny<1, 2>(ctx, g);

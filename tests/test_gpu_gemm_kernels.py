@@ -559,6 +559,13 @@ def test_few_rows_share_k_between_waves(be, rows, k, n):
     assert np.abs(be.download_f32(act) - ref).max() <= 1e-2 * max(1.0, float(np.abs(ref).max()))
 
 
+@pytest.mark.parametrize("rows,k,n", [(1, 128, 1), (4, 128, 4), (2, 768, 1023), (4, 1024, 1024), (3, 1152, 5), (1, 3072, 768), (4, 8192, 77),
+                                      (2, 256, 1025), (5, 3072, 768)])
+def test_few_rows_in_quarters_of_k(be, rows, k, n):
+    """gemm_rows4_kernel (up to four rows, 1024 columns) at its edges: as above."""
+    test_few_rows_share_k_between_waves(be, rows, k, n)
+
+
 @pytest.mark.parametrize("rows,k,n", [(16, 16, 16), (16, 4, 16), (48, 20, 32), (100, 260, 36), (256, 256, 256), (130, 8, 62), (704, 256, 704),
                                       (1030, 72, 260), (52, 3000, 44), (2048, 256, 256), (31, 64, 29)])
 def test_small_f32_outputs_share_k_between_waves(be, rows, k, n):
