@@ -339,152 +339,120 @@ __global__ void fill_positions_kernel(const unsigned int* __restrict__ ids, unsi
   positions[slot] = static_cast<unsigned int>(n);
 }
 
-// fill_positions_kernel leaves a row's token positions in arrival order. The sums below must run
-// in ascending token order (the order of the CPU scatter, pointwise.rs:196-207) to carry the same
-// bits, so every row's segment is sorted first, out of place:
-//   * up to 64 positions: one wave, a bitonic network over lane shuffles;
-//   * longer segments (one id filling a large share of the batch) are queued and sorted by
-//     sort_long_segments_kernel below.
-__global__ __launch_bounds__(ROW_THREADS) void sort_short_segments_kernel(const unsigned int* __restrict__ offsets,
-                                                                          const unsigned int* __restrict__ positions,
-                                                                          unsigned int* __restrict__ sorted,
-                                                                          unsigned int* __restrict__ long_count,
-                                                                          unsigned int* __restrict__ long_rows,
-                                                                          size_t vocab) {
-  const int lane = threadIdx.x & 63;
-  const size_t v = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (v >= vocab) return;
-  const unsigned int begin = offsets[v], end = offsets[v + 1], len = end - begin;
-  if (len == 0) return;
-  if (len > 64) {
-    if (lane == 0) long_rows[atomicAdd(long_count, 1u)] = static_cast<unsigned int>(v);
-    return;
-  }
-  unsigned int p = static_cast<unsigned int>(lane) < len ? positions[begin + lane] : 0xffffffffu;
-#pragma unroll
-  for (int k = 2; k <= 64; k <<= 1)
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const unsigned int other = __shfl_xor(p, j, 64);
-      const bool ascending = (lane & k) == 0;
-      const bool keep_min = ((lane & j) == 0) == ascending;
-      p = keep_min ? min(p, other) : max(p, other);
-    }
-  if (static_cast<unsigned int>(lane) < len) sorted[begin + lane] = p;
-}
-
-// One 1024-thread block per queued row. Positions are distinct token indices, so a bitmap orders
-// them: for each window of 32768 tokens the block marks the row's positions that fall into it
-// (one word per thread), then writes the set bits out in order at a running offset. Linear in
-// the segment's length per window, whatever the length.
-__global__ __launch_bounds__(1024) void sort_long_segments_kernel(const unsigned int* __restrict__ offsets,
-                                                                   const unsigned int* __restrict__ positions,
-                                                                   unsigned int* __restrict__ sorted,
-                                                                   const unsigned int* __restrict__ long_count,
-                                                                   const unsigned int* __restrict__ long_rows,
-                                                                   size_t tokens) {
-  __shared__ unsigned int bitmap[1024];
+// The three in one for a batch and a table that one workgroup's LDS holds the counts of: counts, offsets and positions (2048 tokens
+// in a table of 8192: 5.3 us against five launches of 2.5 to 4.7 each).
+constexpr uint64_t INDEX_TOKENS = 16384, INDEX_VOCAB = 34816;
+__device__ __host__ inline unsigned int index_at(unsigned int i) { return i + (i >> 5); }  // a thread's run of 32 counts: distinct banks
+__global__ __launch_bounds__(1024) void index_ids_kernel(const unsigned int* __restrict__ ids, unsigned int* __restrict__ offsets,
+                                                         unsigned int* __restrict__ positions, unsigned int tokens,
+                                                         unsigned int vocab, OmxFaultWord* fault, unsigned long long tag) {
+  extern __shared__ unsigned int index_counts[];  // [index_at(vocab)]: counts, then where a row's next position goes
   __shared__ unsigned int wave_tot[16];
-  __shared__ unsigned int written;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const unsigned int rows = *long_count;
-  for (unsigned int q = blockIdx.x; q < rows; q += gridDim.x) {
-    const unsigned int v = long_rows[q];
-    const unsigned int begin = offsets[v], end = offsets[v + 1];
-    if (threadIdx.x == 0) written = 0;
-    for (size_t base = 0; base < tokens; base += 32768) {
-      bitmap[threadIdx.x] = 0;
-      __syncthreads();
-      if (written == end - begin) break;  // uniform: read after the barrier, written before the previous one
-      for (unsigned int s = begin + threadIdx.x; s < end; s += 1024) {
-        const size_t rel = static_cast<size_t>(positions[s]) - base;  // wraps far above the window when below it
-        if (rel < 32768) atomicOr(&bitmap[rel >> 5], 1u << (rel & 31));
-      }
-      __syncthreads();
-      unsigned int w = bitmap[threadIdx.x];
-      const unsigned int c = __popc(w);
-      unsigned int incl = c;
+  constexpr int EACH = INDEX_TOKENS / 1024;
+  const unsigned int tid = threadIdx.x;
+  unsigned int id[EACH];  // all in flight at once, and kept for the second pass
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const unsigned int t = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += t;
-      }
-      if (lane == 63) wave_tot[wave] = incl;
-      __syncthreads();
-      unsigned int before = written;
-      for (int wv = 0; wv < wave; ++wv) before += wave_tot[wv];
-      unsigned int at = begin + before + incl - c;
-      while (w) {
-        const int bit = __ffs(w) - 1;
-        sorted[at++] = static_cast<unsigned int>(base) + threadIdx.x * 32 + bit;
-        w &= w - 1;
-      }
-      __syncthreads();
-      if (threadIdx.x == 1023) written = before + incl;
-      __syncthreads();
+  for (int i = 0; i < EACH; ++i)
+    if (i * 1024u < tokens) id[i] = ids[min(tid + i * 1024u, tokens - 1)];
+  for (unsigned int i = tid; i < vocab; i += 1024) index_counts[index_at(i)] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < EACH; ++i)
+    if (tid + i * 1024u < tokens) {
+      if (id[i] >= vocab) dev_raise_range(fault, tag);
+      else atomicAdd(&index_counts[index_at(id[i])], 1u);
     }
-    __syncthreads();
+  __syncthreads();
+  const unsigned int each = (vocab + 1023) / 1024, first = min(vocab, tid * each), last = min(vocab, first + each);
+  unsigned int mine = 0;
+  for (unsigned int i = first; i < last; ++i) mine += index_counts[index_at(i)];
+  unsigned int total;
+  unsigned int at = scan_block_1024(mine, wave_tot, &total);
+  for (unsigned int i = first; i < last; ++i) {
+    const unsigned int c = index_counts[index_at(i)];
+    index_counts[index_at(i)] = at;
+    at += c;
   }
+  __syncthreads();
+  for (unsigned int i = tid; i < vocab; i += 1024) offsets[i] = index_counts[index_at(i)];
+  if (tid == 0) offsets[vocab] = total;
+  __syncthreads();  // (read before the positions move them)
+#pragma unroll
+  for (int i = 0; i < EACH; ++i)
+    if (tid + i * 1024u < tokens && id[i] < vocab) positions[atomicAdd(&index_counts[index_at(id[i])], 1u)] = tid + i * 1024u;
 }
 
-// One wave per table row: zero it, or add its tokens' gradient rows in ascending token order
-// (`sorted`: the row's positions, ascending), so the f32 sums carry the CPU scatter's bits.
+// One wave per table row and columns blockIdx.y, + gridDim.y, ... of 64 x 4 (x 8 of single ones): zero them, or add the row's tokens'
+// gradients in ascending token order, so the f32 sums carry the CPU scatter's bits (pointwise.rs:196-207). `positions` hold a row's
+// tokens in arrival order. Up to 64 are sorted by a bitonic network over the lanes; more, by the whole workgroup, whose waves then take
+// the row's columns in turn: a bitmap of 32768 tokens at a time, its set bits listed 2048 tokens at a time. Bound by the latency of
+// the gradient rows, so eight are in flight (one at a time, 16 tokens each of 1024 rows of 768: 38.7 us, now 12.3 on three times the
+// waves; a bitmap per wave had the empty rows of a large table wait for LDS: 16384 tokens of 50304 rows 54 us, now 36).
 // V = 4: a lane owns four consecutive columns (16-byte accesses; dim a multiple of 4, aligned rows).
 // ADD: the row's sum, complete, is added to what `table_grad` holds (the bits of the scatter
 // followed by accumulate_grad), and rows no token names are left alone.
 template <typename TG, int V, bool ADD>
 __global__ __launch_bounds__(ROW_THREADS) void embedding_bwd_kernel(const unsigned int* __restrict__ offsets,
-                                                                    const unsigned int* __restrict__ sorted,
+                                                                    const unsigned int* __restrict__ positions,
                                                                     const TG* __restrict__ grad,
                                                                     float* __restrict__ table_grad, size_t vocab,
-                                                                    int dim, OmxFaultWord* fault,
+                                                                    int dim, size_t tokens, OmxFaultWord* fault,
                                                                     unsigned long long tag) {
-  const int lane = threadIdx.x & 63;
-  const size_t v = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (v >= vocab) return;
-  const unsigned int begin = offsets[v], end = offsets[v + 1];
-  float* dst = table_grad + v * dim;
-  if (begin == end) {
-    if constexpr (ADD) return;
-    if constexpr (V == 4) {
-      for (int c = lane * 4; c < dim; c += 256) *reinterpret_cast<float4*>(dst + c) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    } else {
-      for (int c = lane; c < dim; c += 64) dst[c] = 0.0f;
-    }
-    return;
-  }
+  constexpr int WINDOW = 32768, GROUP = 2048;  // tokens; a group is a word per lane
+  constexpr unsigned int SHORT = 64;
+  __shared__ unsigned int bitmap[WINDOW / 32];
+  __shared__ unsigned short list[GROUP];
+  __shared__ unsigned int listed;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const size_t v0 = static_cast<size_t>(blockIdx.x) * 4;
+  unsigned int at[5];  // where the four rows' positions start
+#pragma unroll
+  for (int r = 0; r < 5; ++r) at[r] = offsets[min(v0 + r, vocab)];
+  constexpr int CHUNKS = V == 4 ? 1 : 8, COLUMNS = 64 * V * CHUNKS;
   bool bad = false;
-  constexpr int CHUNKS = 8 / V;  // 8 columns per lane and pass
-  for (int c0 = 0; c0 < dim; c0 += 64 * 8) {
-    float acc[CHUNKS][V];
+  float acc[CHUNKS][V];
+  auto clear = [&] {
 #pragma unroll
     for (int j = 0; j < CHUNKS; ++j)
 #pragma unroll
       for (int e = 0; e < V; ++e) acc[j][e] = 0.0f;
-    for (unsigned int s = begin; s < end; ++s) {
-      const TG* src = grad + static_cast<size_t>(sorted[s]) * dim;
+  };
+  // The gradients of tokens p of lanes s .. s + AHEAD - 1, and of lanes 0 .. n - 1, in that order.
+  auto add_some = [&](int c0, unsigned int p, unsigned int s, auto ahead) {
+    constexpr int AHEAD = decltype(ahead)::value;
+    float g[AHEAD][CHUNKS][V];
+#pragma unroll
+    for (int r = 0; r < AHEAD; ++r) {
+      const TG* src = grad + static_cast<size_t>(static_cast<unsigned int>(__builtin_amdgcn_readlane(p, s + r))) * dim;
 #pragma unroll
       for (int j = 0; j < CHUNKS; ++j) {
         const int c = c0 + (j * 64 + lane) * V;
-        if (c < dim) {
-          if constexpr (V == 4) {
-            float g[4];
-            dev_load4<TG>(src, c, g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[j][e] = acc[j][e] + g[e];
-          } else {
-            acc[j][0] = acc[j][0] + dev_load<TG>(src, c);
-          }
-        }
+        if constexpr (V == 4) dev_load4<TG>(src, min(c, dim - 4), g[r][j]);
+        else g[r][j][0] = dev_load<TG>(src, min(c, dim - 1));
       }
     }
+#pragma unroll
+    for (int r = 0; r < AHEAD; ++r)
+#pragma unroll
+      for (int j = 0; j < CHUNKS; ++j)
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[j][e] = acc[j][e] + g[r][j][e];
+  };
+  auto add_rows = [&](int c0, unsigned int p, unsigned int n) {
+    unsigned int s = 0;
+    if constexpr (V == 4)
+      for (; s + 8 <= n; s += 8) add_some(c0, p, s, std::integral_constant<int, 8>());
+    for (; s + 2 <= n; s += 2) add_some(c0, p, s, std::integral_constant<int, 2>());
+    if (s < n) add_some(c0, p, s, std::integral_constant<int, 1>());
+  };
+  auto store = [&](float* dst, int c0, bool add) {
 #pragma unroll
     for (int j = 0; j < CHUNKS; ++j) {
       const int c = c0 + (j * 64 + lane) * V;
       if (c < dim) {
 #pragma unroll
         for (int e = 0; e < V; ++e) bad |= !dev_finite(acc[j][e]);
-        if constexpr (ADD) {
+        if (add) {
           if constexpr (V == 4) {
             const float4 old = *reinterpret_cast<const float4*>(dst + c);
             acc[j][0] = old.x + acc[j][0];
@@ -498,6 +466,63 @@ __global__ __launch_bounds__(ROW_THREADS) void embedding_bwd_kernel(const unsign
         if constexpr (V == 4) *reinterpret_cast<float4*>(dst + c) = make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
         else dst[c] = acc[j][0];
       }
+    }
+  };
+  const size_t v = v0 + wave;
+  const unsigned int begin = wave == 0 ? at[0] : wave == 1 ? at[1] : wave == 2 ? at[2] : at[3];
+  const unsigned int len = (wave == 0 ? at[1] : wave == 1 ? at[2] : wave == 2 ? at[3] : at[4]) - begin;
+  if (v < vocab && len <= SHORT && !(ADD && len == 0)) {
+    unsigned int few = 0xffffffffu;
+    if (static_cast<unsigned int>(lane) < len) few = positions[begin + lane];
+    for (unsigned int k = 2; k >> 1 < len; k <<= 1)
+      for (unsigned int j = k >> 1; j > 0; j >>= 1) {
+        const unsigned int other = __shfl_xor(few, j, 64);
+        const bool ascending = (lane & k) == 0, keep_min = ((lane & j) == 0) == ascending;
+        few = keep_min ? min(few, other) : max(few, other);
+      }
+    for (int c0 = blockIdx.y * COLUMNS; c0 < dim; c0 += gridDim.y * COLUMNS) {
+      clear();
+      add_rows(c0, few, len);
+      store(table_grad + v * dim, c0, ADD);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (at[r + 1] - at[r] <= SHORT) continue;  // (the workgroup's: so are the barriers below)
+    for (int pass0 = blockIdx.y * COLUMNS; pass0 < dim; pass0 += 4 * gridDim.y * COLUMNS) {
+      const int c0 = pass0 + wave * gridDim.y * COLUMNS;
+      clear();
+      unsigned int left = at[r + 1] - at[r];
+      for (size_t base = 0; base < tokens && left > 0; base += WINDOW) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < WINDOW / 32; i += ROW_THREADS) bitmap[i] = 0;
+        __syncthreads();
+        for (unsigned int s = at[r] + threadIdx.x; s < at[r + 1]; s += ROW_THREADS) {
+          const size_t rel = static_cast<size_t>(positions[s]) - base;  // wraps far above the window when below it
+          if (rel < WINDOW) atomicOr(&bitmap[rel >> 5], 1u << (rel & 31));
+        }
+        for (int group = 0; group < WINDOW / GROUP && left > 0; ++group) {
+          __syncthreads();  // the bitmap is whole, the previous list has been read
+          if (wave == 0) {
+            unsigned int w = bitmap[group * 64 + lane], incl = __popc(w);
+            const unsigned int count = incl;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+              const unsigned int t = __shfl_up(incl, off, 64);
+              if (lane >= off) incl += t;
+            }
+            if (lane == 63) listed = incl;
+            for (unsigned int to = incl - count; w; w &= w - 1) list[to++] = static_cast<unsigned short>(lane * 32 + __ffs(w) - 1);
+          }
+          __syncthreads();
+          const unsigned int total = __builtin_amdgcn_readfirstlane(listed);
+          if (c0 < dim)
+            for (unsigned int s = 0; s < total; s += 64)
+              add_rows(c0, static_cast<unsigned int>(base) + group * GROUP + list[min(s + lane, total - 1)], min(64u, total - s));
+          left -= total;
+        }
+      }
+      if (c0 < dim) store(table_grad + (v0 + r) * dim, c0, ADD);
     }
   }
   if (bad) dev_raise_fault(fault, tag);
@@ -840,68 +865,69 @@ static int32_t embedding_backward_impl(omx_ctx* ctx, const void* ids, const void
   if (tokens == 0 || vocab == 0 || dim == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
   if (tokens > 0xfffffffeull || vocab > 0xfffffffeull || dim > 0x7fffffffull)
     return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: axis does not fit in u32", op);
-  // Workspace: counts[V], offsets[V+1], cursor[V], positions[N], sorted[N], the count of rows with
-  // more than 64 tokens (one word, padded to four) and their list (at most N / 65 of them).
+  // Workspace: offsets[V+1], positions[N]; where one workgroup's LDS does not hold the counts also counts[V], cursor[V] and the
+  // scan's totals.
+  const bool small = tokens <= INDEX_TOKENS && vocab <= INDEX_VOCAB;
   const uint64_t scan_blocks = (vocab + 1023) / 1024;
-  uint64_t words = vocab + (vocab + 1) + vocab + tokens + tokens + 4 + (tokens / 64 + 1) + scan_blocks + 4;
+  const uint64_t words = vocab + 1 + tokens + (small ? 0 : 2 * vocab + scan_blocks);
   void* ws = nullptr;
   int32_t rc = omx_workspace(ctx, words * 4, &ws);
   if (rc != OMX_OK) return rc;
-  unsigned int* counts = static_cast<unsigned int*>(ws);
-  unsigned int* offsets = counts + vocab;
-  unsigned int* cursor = offsets + vocab + 1;
-  unsigned int* positions = cursor + vocab;
-  unsigned int* sorted = positions + tokens;
-  unsigned int* long_count = sorted + tokens;
-  unsigned int* long_rows = long_count + 4;
-  unsigned int* scan_totals = long_rows + (tokens / 64 + 1);
+  unsigned int* offsets = static_cast<unsigned int*>(ws);
+  unsigned int* positions = offsets + vocab + 1;
   unsigned long long tag = omx_tag(ctx, F_EMBEDDING_BACKWARD);
-  rc = omx_fill_zero(ctx, counts, vocab * 4);
-  if (rc != OMX_OK) return rc;
-  rc = omx_fill_zero(ctx, long_count, 16);
-  if (rc != OMX_OK) return rc;
   const unsigned int* idp = static_cast<const unsigned int*>(ids);
-  dim3 tgrid(static_cast<unsigned>((tokens + 255) / 256));
   // Bytes: every gradient row read once, every table row written once (rows no token names get
   // zeros); the adding form reads and writes at most one table row per token.
   const double table_rows = add ? 2.0 * static_cast<double>(tokens < vocab ? tokens : vocab) : static_cast<double>(vocab);
   OmxKernelTimer timer(ctx, OMX_K_EMBED_BWD,
                        static_cast<double>(dim) * (static_cast<double>(tokens) * (grad_dtype == OMX_BF16 ? 2.0 : 4.0) +
                                                    table_rows * 4.0));
-  omx_launch_timed(ctx, count_ids_kernel, tgrid, dim3(256), 0, timer.start(), nullptr, idp, counts, tokens, vocab,
-                   ctx->fault, tag);
-  OMX_LAUNCH_CHECK(ctx, "count_ids_kernel");
-  if (scan_blocks > 4 && scan_blocks <= SCAN_MAX_BLOCKS) {
-    const dim3 sgrid(static_cast<unsigned>(scan_blocks));
-    omx_launch(ctx, scan_totals_kernel, sgrid, dim3(1024), 0, counts, scan_totals, vocab);
-    OMX_LAUNCH_CHECK(ctx, "scan_totals_kernel");
-    omx_launch(ctx, scan_blocks_kernel, sgrid, dim3(1024), 0, counts, scan_totals, offsets, cursor, vocab);
-    OMX_LAUNCH_CHECK(ctx, "scan_blocks_kernel");
+  if (small) {
+    const int lds = static_cast<int>((index_at(static_cast<unsigned int>(vocab)) + 1) * 4);
+    if (lds > 64 * 1024)
+      OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&index_ids_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    omx_launch_timed(ctx, index_ids_kernel, dim3(1), dim3(1024), lds, timer.start(), nullptr, idp, offsets, positions,
+                     static_cast<unsigned int>(tokens), static_cast<unsigned int>(vocab), ctx->fault, tag);
+    OMX_LAUNCH_CHECK(ctx, "index_ids_kernel");
   } else {
-    omx_launch(ctx, scan_counts_kernel, dim3(1), dim3(1024), 0, counts, offsets, cursor, vocab);
-    OMX_LAUNCH_CHECK(ctx, "scan_counts_kernel");
+    unsigned int* counts = positions + tokens;
+    unsigned int* cursor = counts + vocab;
+    unsigned int* scan_totals = cursor + vocab;
+    rc = omx_fill_zero(ctx, counts, vocab * 4);
+    if (rc != OMX_OK) return rc;
+    dim3 tgrid(static_cast<unsigned>((tokens + 255) / 256));
+    omx_launch_timed(ctx, count_ids_kernel, tgrid, dim3(256), 0, timer.start(), nullptr, idp, counts, tokens, vocab,
+                     ctx->fault, tag);
+    OMX_LAUNCH_CHECK(ctx, "count_ids_kernel");
+    if (scan_blocks > 4 && scan_blocks <= SCAN_MAX_BLOCKS) {
+      const dim3 sgrid(static_cast<unsigned>(scan_blocks));
+      omx_launch(ctx, scan_totals_kernel, sgrid, dim3(1024), 0, counts, scan_totals, vocab);
+      OMX_LAUNCH_CHECK(ctx, "scan_totals_kernel");
+      omx_launch(ctx, scan_blocks_kernel, sgrid, dim3(1024), 0, counts, scan_totals, offsets, cursor, vocab);
+      OMX_LAUNCH_CHECK(ctx, "scan_blocks_kernel");
+    } else {
+      omx_launch(ctx, scan_counts_kernel, dim3(1), dim3(1024), 0, counts, offsets, cursor, vocab);
+      OMX_LAUNCH_CHECK(ctx, "scan_counts_kernel");
+    }
+    omx_launch(ctx, fill_positions_kernel, tgrid, dim3(256), 0, idp, cursor, positions, tokens, vocab);
+    OMX_LAUNCH_CHECK(ctx, "fill_positions_kernel");
   }
-  omx_launch(ctx, fill_positions_kernel, tgrid, dim3(256), 0, idp, cursor, positions, tokens, vocab);
-  OMX_LAUNCH_CHECK(ctx, "fill_positions_kernel");
-  dim3 vgrid(static_cast<unsigned>((vocab + 3) / 4));
-  omx_launch(ctx, sort_short_segments_kernel, vgrid, dim3(ROW_THREADS), 0, offsets, positions, sorted,
-                     long_count, long_rows, vocab);
-  OMX_LAUNCH_CHECK(ctx, "sort_short_segments_kernel");
-  omx_launch(ctx, sort_long_segments_kernel, dim3(256), dim3(1024), 0, offsets, positions, sorted,
-                     long_count, long_rows, tokens);
-  OMX_LAUNCH_CHECK(ctx, "sort_long_segments_kernel");
   const bool vec4 = dim % 4 == 0 && (reinterpret_cast<uintptr_t>(grad) & 15u) == 0 &&
                     (reinterpret_cast<uintptr_t>(table_grad) & 15u) == 0 && (grad_dtype == OMX_F32 || dim % 8 == 0);
+  // A wave per row; where rows are few, per row and 256 columns.
+  const uint64_t columns = vec4 ? 256 : 512;
+  dim3 vgrid(static_cast<unsigned>((vocab + 3) / 4), vocab <= 4096 ? static_cast<unsigned>(std::min<uint64_t>((dim + columns - 1) / columns, 64)) : 1u);
 #define EMB_BWD(TG_, V_)                                                                                         \
   do {                                                                                                          \
     if (add)                                                                                                    \
       omx_launch_timed(ctx, embedding_bwd_kernel<TG_, V_, true>, vgrid, dim3(ROW_THREADS), 0, nullptr,          \
-                       timer.stop(), offsets, sorted, static_cast<const TG_*>(grad),                            \
-                       static_cast<float*>(table_grad), vocab, static_cast<int>(dim), ctx->fault, tag);         \
+                       timer.stop(), offsets, positions, static_cast<const TG_*>(grad),                            \
+                       static_cast<float*>(table_grad), vocab, static_cast<int>(dim), tokens, ctx->fault, tag); \
     else                                                                                                        \
       omx_launch_timed(ctx, embedding_bwd_kernel<TG_, V_, false>, vgrid, dim3(ROW_THREADS), 0, nullptr,         \
-                       timer.stop(), offsets, sorted, static_cast<const TG_*>(grad),                            \
-                       static_cast<float*>(table_grad), vocab, static_cast<int>(dim), ctx->fault, tag);         \
+                       timer.stop(), offsets, positions, static_cast<const TG_*>(grad),                            \
+                       static_cast<float*>(table_grad), vocab, static_cast<int>(dim), tokens, ctx->fault, tag); \
   } while (0)
   if (grad_dtype == OMX_F32) {
     if (vec4) EMB_BWD(float, 4);

@@ -179,6 +179,36 @@ def test_embedding_backward_with_one_id_filling_the_batch(be, tokens, vocab, dim
 
 
 @pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("tokens,vocab,dim", [(16384, 34816, 8), (16385, 40, 260), (40, 34817, 4), (2048, 1025, 256), (3000, 32003, 16),
+                                              (16384, 1024, 768), (200, 2, 1032), (63, 1, 4), (64, 1, 5), (65, 1, 8), (4097, 2, 520)])
+def test_embedding_backward_with_and_without_one_workgroups_index(be, tokens, vocab, dim, bf16):
+    """Counts in one workgroup's LDS up to its limits and beyond them; segments of 64 and 65 tokens, more than one group of 2048;
+    columns split over the grid and not: the oracle's bits. An id past the table is refused on either path."""
+    from ojas_amd.backend import BF16, OjasError
+
+    print(f"embedding index {tokens} {vocab} {dim} bf16={bf16}", flush=True)
+    r = np.random.default_rng(tokens + vocab)
+    ids = r.integers(0, vocab, tokens, dtype=np.uint32)
+    ids[r.random(tokens) < 0.2] = vocab - 1
+    grad = r.standard_normal((tokens, dim)).astype(np.float32)
+    if bf16:
+        grad = orc.round_bf16(grad)
+    dg = be.upload(grad, BF16) if bf16 else be.upload(grad)
+    want = orc.embedding_backward(ids, grad, vocab)
+    assert np.array_equal(be.download(be.embedding_backward(be.upload(ids), dg, vocab)).view(np.uint32), want.view(np.uint32))
+    base = r.standard_normal((vocab, dim)).astype(np.float32)
+    acc = be.upload(base)
+    be.embedding_backward_accumulate(be.upload(ids), dg, acc)
+    named = np.unique(ids)
+    base[named] = base[named] + want[named]
+    assert np.array_equal(be.download(acc).view(np.uint32), base.view(np.uint32))
+    ids[tokens // 2] = vocab
+    be.embedding_backward(be.upload(ids), dg, vocab)
+    with pytest.raises(OjasError):
+        be.sync()
+
+
+@pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("tokens,vocab,dim", [(12, 10, 8), (257, 500, 64), (1000, 37, 65), (4096, 50304, 768)])
 def test_embedding_backward_accumulate_is_the_scatter_then_the_sum(be, tokens, vocab, dim, bf16):
     """`embedding_backward_accumulate` leaves in the table gradient the bits of `embedding_backward`
