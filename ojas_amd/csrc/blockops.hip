@@ -11,68 +11,9 @@
 //   per_head_sigmoid_gate_*    ojas-cpu/src/pointwise.rs:1395-1470,1678-1781,1853-1894
 //   value_residual_blend_*     ojas-cpu/src/pointwise.rs:2031-2148
 // Trait: ojas-core/src/backend.rs:1151-1163,1674-1686,1860-1920.
-#include "omx_common.h"
+#include "packs.h"
 
 namespace {
-
-constexpr int BK_THREADS = 256;
-constexpr int BK_PACKS = 4;  // packs per thread
-
-// A pack is V consecutive elements: one 16-byte (f32) or 8-byte (bf16) access
-// when V == 4, one element when V == 1.
-template <typename T, int V>
-__device__ __forceinline__ void load_pack(const T* __restrict__ p, size_t pack, float (&v)[V]) {
-  if constexpr (V == 1) {
-    v[0] = dev_load<T>(p, pack);
-  } else if constexpr (sizeof(T) == 4) {
-    float4 q = reinterpret_cast<const float4*>(p)[pack];
-    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-  } else {
-    uint2 q = reinterpret_cast<const uint2*>(p)[pack];
-    v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u);
-    v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
-  }
-}
-template <typename T, int V>
-__device__ __forceinline__ void store_pack(T* __restrict__ p, size_t pack, const float (&v)[V]) {
-  if constexpr (V == 1) {
-    dev_store<T>(p, pack, v[0]);
-  } else if constexpr (sizeof(T) == 4) {
-    reinterpret_cast<float4*>(p)[pack] = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-    uint2 q;
-    q.x = dev_pack_bf16_pair(v[0], v[1]);
-    q.y = dev_pack_bf16_pair(v[2], v[3]);
-    reinterpret_cast<uint2*>(p)[pack] = q;
-  }
-}
-
-// Packs per thread: one up to four blocks per compute unit, two up to eight, BK_PACKS beyond. A few thousand rows were 16 to 176
-// blocks whose threads took their packs one latency after the other (rope over 1024 x 4 x 64 6.3 us on 32 blocks, 3.2 on 128).
-__host__ __device__ inline uint64_t packs_per_thread(uint64_t packs, uint64_t blocks) {
-  return packs <= blocks * BK_THREADS ? 1 : packs <= blocks * (2 * BK_THREADS) ? 2 : BK_PACKS;
-}
-inline dim3 pack_grid(uint64_t packs) {
-  const uint64_t each = packs_per_thread(packs, 1024), per_block = each * BK_THREADS;
-  const uint64_t blocks = (packs + per_block - 1) / per_block;
-  return dim3(static_cast<unsigned>(blocks > 0 ? blocks : 1));
-}
-#define PACK_LOOP(p, packs)                                                                                             \
-  for (size_t span_ = packs_per_thread(packs, gridDim.x) * BK_THREADS, p = blockIdx.x * span_ + threadIdx.x,            \
-              end_ = min(static_cast<size_t>(packs), (blockIdx.x + 1) * span_);                                          \
-       p < end_; p += BK_THREADS)
-// n / d in 32 bits where they allow it (a 64-bit division is some 100 instructions).
-__device__ __forceinline__ size_t quotient(size_t n, size_t d) {
-  return ((n | d) >> 32) == 0 ? static_cast<unsigned>(n) / static_cast<unsigned>(d) : n / d;
-}
-
-// Whether every pointer allows 4-element packs of `esz`-byte elements.
-inline bool packs_of_four(uint64_t n, size_t esz, std::initializer_list<const void*> ptrs) {
-  if (n % 4 != 0) return false;
-  uintptr_t mask = esz * 4 - 1, bits = 0;
-  for (const void* p : ptrs) bits |= reinterpret_cast<uintptr_t>(p);
-  return (bits & mask) == 0;
-}
 
 // sigmoid(u) and 1 - sigmoid(u), both without cancellation.
 __device__ __forceinline__ void sigmoid_pair(float u, float* s, float* rest) {

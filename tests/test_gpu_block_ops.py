@@ -8,6 +8,8 @@ backward equals the recomputing one). Tolerances as in the other parity file:
 f32 tier 1e-5 relative to max(1, max|cpu|); bf16 tier 2e-2 with operands
 rounded to bf16 on both sides.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -633,3 +635,29 @@ def test_norm_backward_of_short_rows(be, rows, dim):
     size = (np.abs(gw) + np.abs(hat) * np.abs(gw * hat).mean(-1, keepdims=True)) * rstd
     assert (np.abs(be.download(gx) - want) <= 16 * 2.0**-24 * size).all()
     assert (np.abs(be.download(gwt) - (g64 * hat).sum(0)) <= 64 * 2.0**-24 * np.abs(g64 * hat).sum(0)).all()
+
+
+@pytest.mark.parametrize("n,offset", [(1, 0), (3, 0), (4, 0), (1021, 0), (1024, 1), (4 * 1024 * 256 + 4, 0), (4 * 1024 * 256 + 5, 0), (8 * 1024 * 256 + 4, 2)])
+def test_elementwise_packs_of_four_and_single(be, n, offset):
+    """Sums, scaling, casts and GELU in packs of four where length and addresses allow them and one at a time where not (`offset`
+    elements into a buffer): the same bits either way."""
+    from ojas_amd.backend import BF16, F32
+
+    r = np.random.default_rng(n)
+    x, y = (r.standard_normal(n + offset).astype(np.float32) for _ in range(2))
+    dx, dy = (be.upload(v) for v in (x, y))
+    at = lambda t, size: C.c_void_p(t.ptr + offset * size)
+    x, y = x[offset:], y[offset:]
+    out, half = be.empty((n + offset,), F32), be.empty((n + offset,), BF16)
+    f32 = C.c_int32(F32)
+    be._check(be._lib.omx_residual_add(be._ctx, at(dx, 4), f32, at(dy, 4), f32, at(out, 4), f32, C.c_uint64(n)))
+    assert np.array_equal(be.download(out)[offset:], x + y)
+    be._check(be._lib.omx_to_bf16(be._ctx, at(dx, 4), at(half, 2), C.c_uint64(n)))
+    assert np.array_equal(be.download_f32(half)[offset:], orc.round_bf16(x))
+    be._check(be._lib.omx_gelu_forward(be._ctx, at(dx, 4), at(out, 4), f32, C.c_uint64(n), C.c_int32(0)))
+    whole = be.download(be.gelu_erf_forward(be.upload(np.concatenate([x, np.zeros(-n % 4, np.float32)]))))[:n]
+    assert np.array_equal(be.download(out)[offset:], whole)
+    be._check(be._lib.omx_accumulate_grad(be._ctx, at(dy, 4), at(dx, 4), C.c_uint64(n)))
+    assert np.array_equal(be.download(dy)[offset:], y + x)
+    be._check(be._lib.omx_scale_grad(be._ctx, at(dx, 4), C.c_float(0.3), C.c_uint64(n)))
+    assert np.array_equal(be.download(dx)[offset:], x * np.float32(0.3))
