@@ -449,6 +449,32 @@ class MiBackend(_native.Methods):
             _native.omx_causal_attention_backward(*head, *tail)
         return gq, gk, gv
 
+    def causal_attention_f32_forward(self, q, k, v, window: Optional[int] = None):
+        """`causal_attention` (ojas-model/src/block.rs:186-199) of the f32 tier over time-major [B, T, heads, D] tensors:
+        (out, lse [B, heads, T]). Head dims 16 / 32 / 64 / 128."""
+        b, t, h, d = q.shape
+        hkv = k.shape[2]
+        if k.shape != (b, t, hkv, d) or v.shape != k.shape:
+            raise OjasError(SHAPE, f"causal_attention_f32_forward: q {q.shape}, k {k.shape}, v {v.shape}")
+        if not (q.dtype == k.dtype == v.dtype == F32):
+            raise OjasError(DTYPE, "causal_attention_f32_forward: operands must be f32")
+        out, lse = self.empty((b, t, h, d), F32), self.empty((b, h, t), F32)
+        _native.omx_causal_attention_f32_forward(self._context, q, h * d, k, v, hkv * d, out, h * d, lse, b, t, h, hkv, d,
+                                                 window or 0)
+        return out, lse
+
+    def causal_attention_f32_backward(self, q, k, v, out, lse, gy, window: Optional[int] = None):
+        b, t, h, d = q.shape
+        hkv = k.shape[2]
+        if k.shape != (b, t, hkv, d) or v.shape != k.shape or out.shape != q.shape or gy.shape != q.shape or lse.shape != (b, h, t):
+            raise OjasError(SHAPE, f"causal_attention_f32_backward: q {q.shape}, k {k.shape}, v {v.shape}, out {out.shape}, gy {gy.shape}")
+        if any(x.dtype != F32 for x in (q, k, v, out, lse, gy)):
+            raise OjasError(DTYPE, "causal_attention_f32_backward: operands must be f32")
+        gq, gk, gv = self.empty(q.shape, F32), self.empty(k.shape, F32), self.empty(v.shape, F32)
+        _native.omx_causal_attention_f32_backward(self._context, q, h * d, k, v, hkv * d, out, gy, h * d, lse, gq, gk, gv, b, t, h,
+                                                  hkv, d, window or 0)
+        return gq, gk, gv
+
     # ---- norms ----
     def rms_norm_forward(self, x, w, eps: float = 1e-6, out_dtype: Optional[int] = None):
         dim = x.shape[-1]

@@ -460,7 +460,7 @@ struct Symbol {
   X(omx_linear_i8_group_forward) X(omx_linear_i8_group_backward_input) X(omx_pack_i8_group)                              \
   X(omx_causal_sdpa_forward) X(omx_causal_sdpa_backward) X(omx_causal_sdpa_backward_recompute)                           \
   X(omx_linear_gelu_forward) X(omx_linear_backward_input_gelu) X(omx_causal_attention_forward)                           \
-  X(omx_causal_attention_backward) X(omx_causal_attention_forward_saving) X(omx_causal_attention_backward_saved)         \
+  X(omx_causal_attention_backward) X(omx_causal_attention_f32_forward) X(omx_causal_attention_f32_backward) X(omx_causal_attention_forward_saving) X(omx_causal_attention_backward_saved)         \
   X(omx_rms_norm_forward) X(omx_rms_norm_backward) X(omx_residual_add_rms_norm_forward)                                  \
   X(omx_rms_norm_backward_residual) X(omx_cross_entropy_mean_forward) X(omx_cross_entropy_mean_forward_static)           \
   X(omx_cross_entropy_mean_backward) X(omx_linear_cross_entropy_mean) X(omx_embedding_forward) X(omx_embedding_backward) \

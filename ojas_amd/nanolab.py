@@ -100,14 +100,42 @@ class NanolabGraph:
         eps, win = s.rms_eps, s.window
         cos, sin = self._rope_tables(T)
         swap = [0, 2, 1, 3]
+        # On the backend itself, sums ride in the op that makes their second term (the same bits) and attention reads its
+        # operands as they lie; a wrapper that tags every op's result takes them one by one.
+        fused = isinstance(be, MiBackend)
+        time_major = fused and D in (16, 32, 64, 128)
+
+        def add_norm(x, y, w):
+            """x + y and its norm."""
+            if fused:
+                return be.residual_add_rms_norm_forward(x, y, w, eps)
+            total = be.residual_add_forward(x, y)
+            return total, be.rms_norm_forward(total, w, eps)
+
+        def norm_backward_onto(g, x, w, gy):
+            """g + the norm's input gradient, and its weight gradient."""
+            if fused:
+                gx, _, gw = be.rms_norm_backward_residual(x, w, gy, g, eps)
+                return gx, gw
+            gt, gw = be.rms_norm_backward(x, w, gy, eps)
+            return be.residual_add_forward(g, gt), gw
+
+        def linear_backward_onto(g, x, w, gy):
+            """g (which is no one else's) + the projection's input gradient, and its weight gradient."""
+            if fused:
+                _, gw = be.linear_backward(x, w, gy, need_gx=False)
+                nout, kin = w.shape
+                return be.gemm(gy, (nout, 1), w, (kin, 1), N, nout, kin, c=g), gw
+            part, gw = be.linear_backward(x, w, gy)
+            return be.residual_add_forward(g, part), gw
 
         # ---- forward (block.rs:218-264) ----
         x = be.embedding_forward(self.p["tok_emb.weight"], ids).reshape(N, d)
         acts = []
         v0 = None
+        h = be.rms_norm_forward(x, self._blk(0, "norm1.weight"), eps)
         for i in range(s.n_layer):
-            a = {"x": x}
-            a["h"] = be.rms_norm_forward(x, self._blk(i, "norm1.weight"), eps)
+            a = {"x": x, "h": h}
             a["q_lin"] = be.linear_forward(a["h"], self._blk(i, "mixer.q_proj.weight")).reshape(B, T, H, D)
             a["k_lin"] = be.linear_forward(a["h"], self._blk(i, "mixer.k_proj.weight")).reshape(B, T, KV, D)
             a["raw_v"] = be.linear_forward(a["h"], self._blk(i, "mixer.v_proj.weight")).reshape(B, T, KV, D)
@@ -120,22 +148,26 @@ class NanolabGraph:
                 v0 = a["raw_v"]
             else:
                 v = be.value_residual_blend_forward(a["raw_v"], v0, self._blk(i, "mixer.vr_lambda"))
-            a["qp"], a["kp"], a["vp"] = be.permute(q, swap), be.permute(k, swap), be.permute(v, swap)
-            a["att"], a["lse"] = be.causal_sdpa_forward(a["qp"], a["kp"], a["vp"], win)
-            a["ap"] = be.permute(a["att"], swap)  # [B, T, H, D]
+            if time_major:
+                a["qp"], a["kp"], a["vp"] = q, k, v
+                a["ap"], a["lse"] = be.causal_attention_f32_forward(q, k, v, win)  # [B, T, H, D]
+            else:
+                a["qp"], a["kp"], a["vp"] = be.permute(q, swap), be.permute(k, swap), be.permute(v, swap)
+                a["att"], a["lse"] = be.causal_sdpa_forward(a["qp"], a["kp"], a["vp"], win)
+                a["ap"] = be.permute(a["att"], swap)  # [B, T, H, D]
             a["y"], a["scales"] = be.per_head_sigmoid_gate_forward_saving(
                 a["h"].reshape(B, T, d), self._blk(i, "mixer.gate.weight"), self._blk(i, "mixer.gate.bias"), a["ap"])
             o = be.linear_forward(a["y"].reshape(N, H * D), self._blk(i, "mixer.o_proj.weight"))
-            a["x1"] = be.residual_add_forward(x, o)
-            a["h2"] = be.rms_norm_forward(a["x1"], self._blk(i, "norm2.weight"), eps)
+            a["x1"], a["h2"] = add_norm(x, o, self._blk(i, "norm2.weight"))
             a["g_lin"] = be.linear_forward(a["h2"], self._blk(i, "ffn.gate.weight"))
             a["g_act"] = be.silu_forward(a["g_lin"])
             a["up"] = be.linear_forward(a["h2"], self._blk(i, "ffn.up.weight"))
             a["m"] = be.mul_forward(a["g_act"], a["up"])
             down = be.linear_forward(a["m"], self._blk(i, "ffn.down.weight"))
-            x = be.residual_add_forward(a["x1"], down)
+            after = self._blk(i + 1, "norm1.weight") if i + 1 < s.n_layer else self.p["norm_f.weight"]
+            x, h = add_norm(a["x1"], down, after)
             acts.append(a)
-        hf = be.rms_norm_forward(x, self.p["norm_f.weight"], eps)
+        hf = h
         logits = be.linear_forward(hf, self.p["tok_emb.weight"]) if want_logits else None
         tflat = targets.reshape(N)
         loss, ghf, g_head = be.linear_cross_entropy_mean(hf, self.p["tok_emb.weight"], tflat)
@@ -153,11 +185,9 @@ class NanolabGraph:
             g_gact, g_up = be.mul_backward(a["g_act"], a["up"], gm)
             gh2, grads[f"blocks.{i}.ffn.up.weight"] = be.linear_backward(a["h2"], self._blk(i, "ffn.up.weight"), g_up)
             g_glin = be.silu_backward(a["g_lin"], g_gact)
-            part, grads[f"blocks.{i}.ffn.gate.weight"] = be.linear_backward(a["h2"], self._blk(i, "ffn.gate.weight"),
-                                                                           g_glin)
-            gh2 = be.residual_add_forward(gh2, part)
-            gt, grads[f"blocks.{i}.norm2.weight"] = be.rms_norm_backward(a["x1"], self._blk(i, "norm2.weight"), gh2, eps)
-            gx1 = be.residual_add_forward(gx, gt)
+            gh2, grads[f"blocks.{i}.ffn.gate.weight"] = linear_backward_onto(gh2, a["h2"], self._blk(i, "ffn.gate.weight"),
+                                                                             g_glin)
+            gx1, grads[f"blocks.{i}.norm2.weight"] = norm_backward_onto(gx, a["x1"], self._blk(i, "norm2.weight"), gh2)
             gy, grads[f"blocks.{i}.mixer.o_proj.weight"] = be.linear_backward(
                 a["y"].reshape(N, H * D), self._blk(i, "mixer.o_proj.weight"), gx1)
             gh, grads[f"blocks.{i}.mixer.gate.weight"], grads[f"blocks.{i}.mixer.gate.bias"], gap = \
@@ -165,9 +195,12 @@ class NanolabGraph:
                                                         self._blk(i, "mixer.gate.bias"), a["ap"],
                                                         gy.reshape(B, T, H, D), a["scales"])
             gh = gh.reshape(N, d)
-            ga = be.permute(gap, swap)
-            gqp, gkp, gvp = be.causal_sdpa_backward(a["qp"], a["kp"], a["vp"], a["att"], a["lse"], ga, win)
-            gv, gk, gq = be.permute(gvp, swap), be.permute(gkp, swap), be.permute(gqp, swap)
+            if time_major:
+                gq, gk, gv = be.causal_attention_f32_backward(a["qp"], a["kp"], a["vp"], a["ap"], a["lse"], gap, win)
+            else:
+                ga = be.permute(gap, swap)
+                gqp, gkp, gvp = be.causal_sdpa_backward(a["qp"], a["kp"], a["vp"], a["att"], a["lse"], ga, win)
+                gv, gk, gq = be.permute(gvp, swap), be.permute(gkp, swap), be.permute(gqp, swap)
             if i == 0:
                 g_raw_v = gv if g_v0 is None else be.residual_add_forward(g_v0, gv)
                 grads["blocks.0.mixer.vr_lambda"] = be.zeros((1,), F32)
@@ -182,11 +215,9 @@ class NanolabGraph:
                                         self._blk(i, "mixer.k_norm.weight"), gqn, gkn, eps)
             for name, g_out in (("v_proj", g_raw_v.reshape(N, KV * D)), ("k_proj", gk_lin.reshape(N, KV * D)),
                                 ("q_proj", gq_lin.reshape(N, H * D))):
-                part, grads[f"blocks.{i}.mixer.{name}.weight"] = be.linear_backward(
-                    a["h"], self._blk(i, f"mixer.{name}.weight"), g_out)
-                gh = be.residual_add_forward(gh, part)
-            gt, grads[f"blocks.{i}.norm1.weight"] = be.rms_norm_backward(a["x"], self._blk(i, "norm1.weight"), gh, eps)
-            gx = be.residual_add_forward(gx1, gt)
+                gh, grads[f"blocks.{i}.mixer.{name}.weight"] = linear_backward_onto(
+                    gh, a["h"], self._blk(i, f"mixer.{name}.weight"), g_out)
+            gx, grads[f"blocks.{i}.norm1.weight"] = norm_backward_onto(gx1, a["x"], self._blk(i, "norm1.weight"), gh)
         # The tied table: the head's gradient first, then the embedding's rows.
         g_emb = be.embedding_backward(ids.reshape(N), gx, s.vocab)
         grads["tok_emb.weight"] = be.residual_add_forward(g_head, g_emb)

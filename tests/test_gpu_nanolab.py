@@ -58,6 +58,33 @@ def run(be, spec, host_params, ids, targets, want_logits=False):
             {n: be.download(g) for n, g in grads.items()})
 
 
+class OneByOne:
+    """The backend behind a wrapper: the graph then takes every sum and permute as an op of its own."""
+
+    def __init__(self, be):
+        self._be = be
+
+    def __getattr__(self, name):
+        return getattr(self._be, name)
+
+
+@pytest.mark.parametrize("time,heads,kv_heads,dim,window", [(33, 4, 2, 64, None), (40, 2, 2, 16, 9), (17, 3, 1, 24, None)])
+def test_sums_inside_ops_and_attention_in_place_change_nothing(be, time, heads, kv_heads, dim, window):
+    """The graph on the backend against the same graph op by op: an op that adds adds the rounded term (1e-6 of the norm: a
+    product whose reduction is split may add in another order). Head dim 24 keeps the permutes."""
+    from ojas_amd.nanolab import NanolabSpec
+
+    spec = NanolabSpec(n_layer=3, n_embd=96, n_head=heads, n_kv_head=kv_heads, head_dim=dim, hidden=200, vocab=64, window=window)
+    r = np.random.default_rng(time)
+    host = {n: (r.standard_normal(shape) * 0.1 + (1.0 if "norm" in n else 0.0)).astype(np.float32) for n, shape in spec.param_shapes().items()}
+    ids, targets = (r.integers(0, 64, (2, time)) for _ in range(2))
+    loss, _, grads = run(be, spec, host, ids, targets)
+    want_loss, _, want = run(OneByOne(be), spec, host, ids, targets)
+    assert abs(loss - want_loss) <= 1e-6 * abs(want_loss)
+    for name in want:
+        assert np.linalg.norm(grads[name] - want[name]) <= 1e-6 * max(np.linalg.norm(want[name]), 1e-6), name
+
+
 def test_tiny_fixture_forward_and_gradients(be):
     print("nanolab tiny fixture on the device", flush=True)
     spec = tiny_spec()
