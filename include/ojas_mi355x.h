@@ -675,7 +675,7 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * LDS-tiled kernel. "ce_fused": 0 = the fused linear-cross-entropy always takes its separate
  * statistics and gradient kernels (default 1: one kernel when a tile holds the whole
  * vocabulary). "adamw_trust": 0 = omx_adamw_step_bounded always runs its checking pass
- * (default 1). "muon_fused_sums": 0 = the bf16 Newton-Schulz iteration forms b A + c A^2 and
+ * (default 1). "muon_fused_sums": 0 = the Newton-Schulz iteration forms b A + c A^2 and
  * a X + B X in kernels of their own instead of in the products' store passes (default 1; the
  * same bits either way). "sdpa_tiled": 0 = f32 attention always takes the one-wave-per-row
  * kernels (default 1: matrix-unit kernels at head_dim 16 / 32 / 64 / 128 with 16-byte aligned

@@ -358,8 +358,9 @@ __global__ void splitk_reduce_kernel(GemmArgs g) {
        i += static_cast<long>(gridDim.x) * blockDim.x) {
     const long row = i / g.N, col = i - row * g.N;
     const long off = row * g.ldc + col;
-    float acc = g.accumulate ? static_cast<float*>(g.c)[off] : 0.0f;
+    float acc = g.accumulate == 1 ? static_cast<float*>(g.c)[off] : 0.0f;
     for (int s = 0; s < g.splits; ++s) acc += g.partial[static_cast<long>(s) * total + i];
+    if (g.accumulate == 2) acc = gemm_add32(g, reinterpret_cast<const float*>(g.aux_in)[off], acc);
     if (g.c_bf16) static_cast<unsigned short*>(g.c)[off] = dev_f32_to_bf16_bits(acc);
     else static_cast<float*>(g.c)[off] = acc;
     bad |= !dev_finite(acc);
@@ -511,6 +512,9 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   const char* op = omx_fault_name(fault_op);
   const uint64_t batches = batch ? batch->count : 1;
   if (batches == 0 || batches > 65535) return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: 1..65535 products per launch", op);
+  // A two-term sum in f32 is accumulation from another tensor: any f32 kernel takes it, a split reduction's last pass too.
+  const OmxGemmEpilogue* sum32 = epi && epi->mode == OMX_EPI_AXPBY && operand_dtype == OMX_F32 && c_dtype == OMX_F32 ? epi : nullptr;
+  if (sum32) epi = nullptr;
   if (epi && epi->mode != OMX_EPI_NONE && c_dtype != OMX_BF16)
     return omx_fail(ctx, OMX_DTYPE, "%s: a fused activation needs a bf16 output", op);
   if (!a || !b || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
@@ -553,7 +557,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   g.K = g.k_rows = static_cast<int>(k);
   g.a_k = a_k > k && a_k <= 0x7fffffffull ? static_cast<int>(a_k) : g.K;
   g.c_bf16 = c_dtype == OMX_BF16;
-  g.accumulate = accumulate;
+  g.accumulate = sum32 ? 2 : accumulate;
   g.a_vec = aligned16(a) && (lda % kv == 0);
   g.b_vec = aligned16(b) && (ldb % kv == 0);
   g.c_vec = aligned16(c) && (ldc % 4 == 0);
@@ -810,6 +814,12 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   g.epi_s1 = epi ? epi->s1 : 0.0f;
   g.epi_s2 = epi ? epi->s2 : 0.0f;
   // The activation's side tensor is accessed with the output's vector width.
+  if (sum32) {
+    g.aux_in = static_cast<const unsigned short*>(sum32->aux_in);
+    g.epi_s1 = sum32->s1;
+    g.epi_s2 = sum32->s2;
+    if (!aligned16(sum32->aux_in)) g.c_vec = 0;
+  }
   if (epi && !((!epi->aux_in || aligned16(epi->aux_in)) && (!epi->aux_out || aligned16(epi->aux_out)))) g.c_vec = 0;
   g.fault = ctx->fault;
   g.tag = omx_tag(ctx, fault_op);

@@ -11,7 +11,7 @@ struct GemmArgs {
   int M, N, K;
   int k_rows;  // direct-to-LDS kernels: K is rounded up to whole steps, k-major operands end after k_rows rows
   int a_k;     // columns of a k-contiguous A's rows that may be read (zeros past K); K itself otherwise
-  int c_bf16, accumulate;
+  int c_bf16, accumulate;  // accumulate 2 (f32 output): C = epi_s1 * aux_in (as f32) + epi_s2 * A.B
   int a_vec, b_vec;  // 16-byte loads allowed (alignment of base and leading dimension)
   int c_vec;         // 4-column stores allowed (alignment of C and its row pitch)
   int tiles_m, tiles_n;
@@ -42,6 +42,11 @@ __device__ __forceinline__ void gemm_select_batch(GemmArgs& g, int product) {
     if (g.aux_in) g.aux_in = reinterpret_cast<const unsigned short*>(reinterpret_cast<const char*>(g.aux_in) + y * g.batch_c);
     if (g.aux_out) g.aux_out = reinterpret_cast<unsigned short*>(reinterpret_cast<char*>(g.aux_out) + y * g.batch_c);
   }
+}
+
+// What an accumulating f32 product stores: `old` is C's value, or aux_in's (accumulate 2).
+__device__ __forceinline__ float gemm_add32(const GemmArgs& g, float old, float acc) {
+  return g.accumulate == 2 ? g.epi_s1 * old + g.epi_s2 * acc : acc + old;
 }
 
 // Stores four consecutive columns of one output row (row `grow`, columns
@@ -79,19 +84,20 @@ __device__ __forceinline__ bool gemm_store4(const GemmArgs& g, int split, int gr
     }
   } else {
     float* cp = static_cast<float*>(g.c) + off;
+    const float* ap = g.accumulate == 2 ? reinterpret_cast<const float*>(g.aux_in) + off : cp;
     if (whole) {
       if (g.accumulate) {
-        const float4 old = *reinterpret_cast<const float4*>(cp);
-        x[0] += old.x;
-        x[1] += old.y;
-        x[2] += old.z;
-        x[3] += old.w;
+        const float4 old = *reinterpret_cast<const float4*>(ap);
+        x[0] = gemm_add32(g, old.x, x[0]);
+        x[1] = gemm_add32(g, old.y, x[1]);
+        x[2] = gemm_add32(g, old.z, x[2]);
+        x[3] = gemm_add32(g, old.w, x[3]);
       }
       *reinterpret_cast<float4*>(cp) = make_float4(x[0], x[1], x[2], x[3]);
       bad = !(dev_finite(x[0]) && dev_finite(x[1]) && dev_finite(x[2]) && dev_finite(x[3]));
     } else {
       for (int e = 0; e < 4 && gcol + e < g.N; ++e) {
-        float y = g.accumulate ? x[e] + cp[e] : x[e];
+        float y = g.accumulate ? gemm_add32(g, ap[e], x[e]) : x[e];
         cp[e] = y;
         bad |= !dev_finite(y);
       }

@@ -265,11 +265,11 @@ int32_t run_muon(omx_ctx* ctx, const MuonTensors& t, unsigned count, uint64_t ro
   const OmxGemmBatch* bp = count > 1 ? &batch : nullptr;
   TX* am = reinterpret_cast<TX*>(ws + L.a);
   TX* a2 = reinterpret_cast<TX*>(ws + L.a2);
-  // bf16 tier: the two-term sums after the second and third product ride in those products' store
-  // passes (the same roundings in the same order as the combine kernels below; a non-finite value
-  // raises the fault there and reaches the final check through the remaining products). Strided
-  // batches only: a single product may split its reduction, which a store-pass sum cannot follow.
-  const bool fused = sizeof(TX) == 2 && s.bf16 && ctx->muon_fused_sums && count > 1;
+  // The two-term sums after the second and third product ride in those products' store passes (the same roundings in the same
+  // order as the combine kernels below; a non-finite value raises the fault there and reaches the final check through the remaining
+  // products). bf16 tier: strided batches only, since a single product may split its reduction, which its store-pass sum cannot
+  // follow. f32: the sums were 46 launches of 3 to 5 us in a step over five shapes.
+  const bool fused = ctx->muon_fused_sums && (sizeof(TX) == 2 ? s.bf16 && count > 1 : !s.bf16);
   for (int it = 0; it < 5; ++it) {
     TX* x = reinterpret_cast<TX*>(ws + x_off);
     TX* xn = reinterpret_cast<TX*>(ws + xn_off);

@@ -104,7 +104,7 @@ struct omx_ctx {
   int adamw_trust = 1;        // 0: omx_adamw_step_bounded always runs its checking pass
   int ce_fused = 1;           // 0: linear-CE always takes the separate statistics and gradient kernels
   int sdpa_tiled = 1;         // 0: f32 attention always takes the one-wave-per-row kernels
-  int muon_fused_sums = 1;    // 0: Newton-Schulz forms b A + c A^2 and a X + B X in kernels of their own (bf16 tier)
+  int muon_fused_sums = 1;    // 0: Newton-Schulz forms b A + c A^2 and a X + B X in kernels of their own
   bool profile_gemm = false;
   uint32_t profile_classes = 0;  // bit per OmxKernelClass other than the products (omx_profile_kernels)
   // The events of the product being launched (null when not timing): the first kernel of the
@@ -187,7 +187,8 @@ inline unsigned long long omx_tag(omx_ctx* ctx, uint32_t op) {
 //   OMX_EPI_GELU_FWD: C = u (rounded to bf16) and aux_out = gelu(u);
 //   OMX_EPI_GELU_BWD: C = round_bf16(A.B) * gelu'(aux_in);
 //   OMX_EPI_AXPBY: C = round_bf16(s1 aux_in) + round_bf16(s2 round_bf16(A.B)): the product stored as
-//     bf16, then the two-term sum a separate pass over it would form, in one store.
+//     bf16, then the two-term sum a separate pass over it would form, in one store. f32 operands and output: C = s1 aux_in +
+//     s2 A.B, each term rounded as a pass of its own would.
 // aux tensors have C's layout (pitch, and batch stride in a strided batch).
 enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3 };
 struct OmxGemmEpilogue {

@@ -247,3 +247,37 @@ def test_a_model_of_many_matrices_steps_within_its_budget():
     assert np.isfinite(tr.run([(ids, ids)], 0.1).loss)
     del tr
     be.close()
+
+
+@pytest.mark.parametrize("rows,cols,count", [(1, 5, 1), (63, 48, 2), (130, 70, 3), (256, 704, 8), (704, 256, 4), (64, 256, 8), (768, 768, 1),
+                                             (1024, 300, 1), (2000, 90, 1)])
+def test_f32_iteration_sums_in_the_store_pass_carry_the_separate_kernels_bits(be, rows, cols, count):
+    """The same of the f32 iteration, a single tensor's split reductions (whose last pass adds) and odd widths included."""
+    from ojas_amd.backend import NON_FINITE, MuonNs5Config, OjasError
+
+    print(f"muon f32 fused sums {count} x {rows}x{cols}", flush=True)
+    r = np.random.default_rng(rows + 3 * cols + count)
+    ps, gs, ms = ([(r.standard_normal((rows, cols)) * size).astype(np.float32) for _ in range(count)] for size in (0.1, 0.03, 0.01))
+    cfg = MuonNs5Config(0.02, 0.95, 0.1, 1, 0)
+    got = {}
+    try:
+        for fused in (1, 0):
+            be.set_option("muon_fused_sums", fused)
+            dp, dg, dm = ([be.upload(x) for x in xs] for xs in (ps, gs, ms))
+            be.muon_ns5_step_batched(dp, dg, dm, cfg, None)
+            be.sync()
+            got[fused] = [be.download(t) for t in dp + dm]
+            bad = [g.copy() for g in gs]
+            bad[-1][rows // 2, cols // 3] = np.inf
+            dp, dg, dm = ([be.upload(x) for x in xs] for xs in (ps, bad, ms))
+            be.muon_ns5_step_batched(dp, dg, dm, cfg, None)
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.code == NON_FINITE and "muon" in e.value.detail
+            for t, want in zip(dp + dm, ps + ms):
+                assert np.array_equal(be.download(t), want)
+    finally:
+        be.set_option("muon_fused_sums", 1)
+    for a, b in zip(got[1], got[0]):
+        assert np.array_equal(a, b)
+    assert any(np.any(a != p) for a, p in zip(got[1][:count], ps))
