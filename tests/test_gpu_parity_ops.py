@@ -1068,7 +1068,7 @@ def test_causal_sdpa_backward_reads_out_and_grad_output_in_their_own_dtypes(be, 
         close(be.download(a), og, F32_TOL, "f32 recompute")
 
 
-@pytest.mark.parametrize("cols", [1, 3, 64, 255, 257, 4096, 4099, 50257])
+@pytest.mark.parametrize("cols", [1, 3, 64, 255, 257, 4096, 4099, 16383, 16384, 16389, 50257])
 def test_argmax_of_rows_at_every_alignment(be, cols):
     """Rows that start off a 16-byte boundary, each workgroup size, a tie that the lowest column wins."""
     x = np.random.default_rng(cols).standard_normal((5, cols)).astype(np.float32)
