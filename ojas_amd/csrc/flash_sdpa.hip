@@ -1194,7 +1194,10 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
   // the chip's workgroup places.
   const unsigned q_blocks = static_cast<unsigned>((s.time + 127) / 128), planes = static_cast<unsigned>(s.batch * s.heads);
   const int tiles = flash_tiles(s);
-  const int groups = flash_groups(ctx, planes, s.time, tiles, s.window > 0, D);
+  // Head dim 128: from 12 tiles on. Over fewer, two groups gain 0.4 to 4 us (16 heads x 128 / 512: 8.4 -> 8.0, 18.8 -> 14.6), and while
+  // their error against 64 bits is 4 % smaller, the probabilities round elsewhere: the worst adapter gradient of two wide blocks over
+  // 512 tokens went from 0.0185 to 0.0200 of its tensor's largest value, where 0.02 is asked for.
+  const int groups = D == 128 && tiles < 12 && ctx->flash_schedule == 0 ? 1 : flash_groups(ctx, planes, s.time, tiles, s.window > 0, D);
   s.q_single = groups > 1 || flash_single(ctx, (q_blocks + 1) / 2 * planes, D == 64 ? 3 : 2, false);
   const unsigned rows = 128 / groups;
   dim3 grid((s.q_single ? (s.time + rows - 1) / rows : (q_blocks + 1) / 2) * planes), block(FT);
