@@ -36,7 +36,7 @@
 // On vector instructions, through shared tiles and now, us, forward / backward (batch x heads over KV heads x time x head
 // dim): 8 x 4/4 x 256 x 64: 38 / 109, 13 / 34, 11 / 30; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370, 20 / 66, 19 / 60; 16 x 12/12
 // x 512 x 64 (shared tiles still): 272 / 1337, 132 / 439 (48 and 37 TFLOP/s, causal-counted); 16 x 4096 x 64: 587 / 1868 through shared
-// tiles, 325 / 1120; 1 x 2/1 x 3000 x 128: 696 / 3334, 151 / 409, 85 / 269.
+// tiles, 325 / 1120; 1 x 2/1 x 3000 x 128: 696 / 3334, 151 / 409, 86 / 216.
 #include <algorithm>
 #include <cmath>
 
@@ -1285,11 +1285,22 @@ int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
   }
   const bool narrow = at_narrow(ctx, a, planes, a.tk, at_span(a) * a.rep);
   const long bk = narrow ? 16 : 64, blocks = (a.tk + bk - 1) / bk;
-  // Split the rows until there are two workgroups per compute unit, as long as a share keeps two tiles of 64 (a part
-  // costs its write, its read and a launch).
+  // Into how many parts the rows are split: two workgroups per compute unit or more, as long as a share keeps two tiles of 64. Under the
+  // causal mask, where the first keys' workgroups are the longest, more where that is less of: their steps, 0.8 us each at head_dim 64,
+  // 0.45 times for each workgroup of a compute unit (the longest go out first, the shorter ones fill in), and for parts a second launch
+  // with their write and read. (In a window all are as long: 57 us with two parts, 61 with four over 777 in 256. One is 54, but a
+  // part's sum is a chain, and one chain's error against 64 bits was 13 % larger.) Backward, us, without the second rule / now:
+  // 8 heads over 2 x 777, batch 2: 89 / 74; 8 over 4 x 777 x 128: 152 / 130; 4 over 1 x 2048: 132 / 121; 2 over 1 x 3000 x 128: 270 / 216.
   const long seen = a.window > 0 ? std::min<long>(a.tk, a.window + bk) : a.tk;
-  const long tiles = std::max<long>(1, seen * a.rep / AT_ROWS);
-  long parts = std::max<long>(1, std::min<long>(2l * ctx->cu_count / (planes * blocks), tiles / 2));
+  const long tiles = std::max<long>(1, seen * a.rep / AT_ROWS), units = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  auto cost = [&](long p) {
+    const double shared = std::max(1.0, 0.45 * static_cast<double>(planes * blocks * p) / static_cast<double>(units));
+    return 0.0125 * D * static_cast<double>((tiles + p - 1) / p) * shared + (p > 1 ? 3.0 + 0.5 * static_cast<double>(p) : 0.0);
+  };
+  long parts = std::max<long>(1, std::min<long>(2l * units / (planes * blocks), tiles / 2));
+  if (a.window <= 0 || a.window >= a.tk)
+    for (long p = parts + 1; p <= std::min(tiles / 2, 64l); ++p)
+      if (cost(p) < cost(parts)) parts = p;
   const long total = static_cast<long>(planes) * a.tk * D;
   while (parts > 1 && parts * total * 8 > (256l << 20)) --parts;
   if (parts > 1) {
