@@ -237,6 +237,13 @@ int32_t omx_linear_backward_input_gelu(omx_ctx* ctx, const void* w, const void* 
                                        uint64_t rows, uint64_t in_features, uint64_t out_features,
                                        int32_t tanh_form);
 
+/* The same in f32 throughout: u = x w^T and act = gelu(u); gu = (gy w) gelu'(u). u, act and gu must not overlap an operand. */
+int32_t omx_linear_gelu_f32_forward(omx_ctx* ctx, const void* x, const void* w, void* u, void* act, uint64_t rows,
+                                    uint64_t in_features, uint64_t out_features, int32_t tanh_form);
+int32_t omx_linear_backward_input_gelu_f32(omx_ctx* ctx, const void* w, const void* gy, const void* u, void* gu,
+                                           uint64_t rows, uint64_t in_features, uint64_t out_features,
+                                           int32_t tanh_form);
+
 /* ---- causal_attention (ojas-model/src/block.rs:186-199): permute [0,2,1,3],
  *      causal_sdpa, permute back, done in one pass over time-major tensors.
  *      q / out / gy / gq are [batch, time, heads, head_dim], k / v / gk / gv

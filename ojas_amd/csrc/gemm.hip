@@ -514,7 +514,10 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   if (batches == 0 || batches > 65535) return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: 1..65535 products per launch", op);
   // A two-term sum in f32 is accumulation from another tensor: any f32 kernel takes it, a split reduction's last pass too.
   const OmxGemmEpilogue* sum32 = epi && epi->mode == OMX_EPI_AXPBY && operand_dtype == OMX_F32 && c_dtype == OMX_F32 ? epi : nullptr;
-  if (sum32) epi = nullptr;
+  // GELU in f32: in the store pass of the kernels that have one (gemm_dma32_kernel, A k-contiguous), else a pass of its own after it.
+  const OmxGemmEpilogue* act32 = epi && (epi->mode == OMX_EPI_GELU_FWD || epi->mode == OMX_EPI_GELU_BWD) && operand_dtype == OMX_F32 &&
+                                         c_dtype == OMX_F32 && !accumulate && batches == 1 && ldc == n ? epi : nullptr;
+  if (sum32 || act32) epi = nullptr;
   if (epi && epi->mode != OMX_EPI_NONE && c_dtype != OMX_BF16)
     return omx_fail(ctx, OMX_DTYPE, "%s: a fused activation needs a bf16 output", op);
   if (!a || !b || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
@@ -821,6 +824,14 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     if (!aligned16(sum32->aux_in)) g.c_vec = 0;
   }
   if (epi && !((!epi->aux_in || aligned16(epi->aux_in)) && (!epi->aux_out || aligned16(epi->aux_out)))) g.c_vec = 0;
+  const bool act_fused = act32 && dma32 >= 0 && !a_km && g.splits == 1;
+  if (act_fused) {
+    g.epi = act32->mode;
+    g.epi_tanh = act32->tanh_form;
+    g.aux_in = static_cast<const unsigned short*>(act32->aux_in);
+    g.aux_out = static_cast<unsigned short*>(act32->aux_out);
+    if (!aligned16(act32->mode == OMX_EPI_GELU_FWD ? act32->aux_out : act32->aux_in)) g.c_vec = 0;
+  }
   g.fault = ctx->fault;
   g.tag = omx_tag(ctx, fault_op);
   omx_ctx::TimedLaunch timed{};
@@ -867,6 +878,9 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     ctx->timing_start = ctx->timing_stop = nullptr;
     if (rc == OMX_OK) ctx->timed.push_back(timed);
   }
+  if (rc == OMX_OK && act32 && !act_fused)
+    rc = act32->mode == OMX_EPI_GELU_FWD ? omx_gelu_forward(ctx, c, act32->aux_out, OMX_F32, m * n, act32->tanh_form)
+                                         : omx_gelu_backward(ctx, act32->aux_in, c, c, OMX_F32, m * n, act32->tanh_form);
   return rc;
 }
 

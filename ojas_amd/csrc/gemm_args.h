@@ -106,6 +106,38 @@ __device__ __forceinline__ bool gemm_store4(const GemmArgs& g, int split, int gr
   return bad;
 }
 
+// The f32 product with its activation: C = the value and aux_out = GELU of it, or C = the value times GELU' of aux_in (f32 all, C's
+// layout), as a pass of its own over the stored product would form them.
+template <bool TANH>
+__device__ __forceinline__ bool gemm_store4_act32(const GemmArgs& g, int grow, int gcol, float x0, float x1, float x2, float x3) {
+  const long off = static_cast<long>(grow) * g.ldc + gcol;
+  float x[4] = {x0, x1, x2, x3};
+  const int n = min(4, g.N - gcol);
+  const bool whole = g.c_vec != 0 && n == 4;
+  bool bad = false;
+  if (g.epi == OMX_EPI_GELU_FWD) {
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[e] = dev_gelu_of<float, TANH>(x[e]);
+      if (e < n) bad |= !dev_finite(y[e]);
+    }
+    float* to = reinterpret_cast<float*>(g.aux_out) + off;
+    if (whole) *reinterpret_cast<float4*>(to) = make_float4(y[0], y[1], y[2], y[3]);
+    else
+      for (int e = 0; e < n; ++e) to[e] = y[e];
+  } else {
+    const float* u = reinterpret_cast<const float*>(g.aux_in) + off;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (whole) dev_load4<float>(u, 0, v);
+    else
+      for (int e = 0; e < n; ++e) v[e] = u[e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = x[e] * dev_gelu_grad_of<float, TANH>(v[e]);
+  }
+  return gemm_store4(g, 0, grow, gcol, x[0], x[1], x[2], x[3]) || bad;
+}
+
 // gemm_store4 with the optional activation of OmxGemmEpilogue applied first (bf16 outputs, no
 // split). Kept apart from the plain store so the plain epilogue loops stay small enough to unroll.
 // OMX_EPI_AXPBY on one element: `aux` as stored, `acc` the product's f32 accumulator.

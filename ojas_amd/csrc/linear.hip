@@ -115,4 +115,26 @@ int32_t omx_linear_backward_input_gelu(omx_ctx* ctx, const void* w, const void* 
                        in_features, rows, out_features, in_features, 0, &epi);
 }
 
+// The f32 tier's forms of the two: the same bits as the product and a pass over it.
+int32_t omx_linear_gelu_f32_forward(omx_ctx* ctx, const void* x, const void* w, void* u, void* act, uint64_t rows, uint64_t in_features,
+                                    uint64_t out_features, int32_t tanh_form) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "linear_gelu_f32_forward";
+  if (!x || !w || !u || !act) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (rows == 0 || in_features == 0 || out_features == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
+  OmxGemmEpilogue epi = {OMX_EPI_GELU_FWD, tanh_form ? 1 : 0, nullptr, act};
+  return omx_gemm_impl(ctx, F_LINEAR_FORWARD, x, in_features, 1, w, 1, in_features, OMX_F32, u, OMX_F32, out_features, rows, in_features,
+                       out_features, 0, &epi);
+}
+int32_t omx_linear_backward_input_gelu_f32(omx_ctx* ctx, const void* w, const void* gy, const void* u, void* gu, uint64_t rows,
+                                           uint64_t in_features, uint64_t out_features, int32_t tanh_form) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "linear_backward_input_gelu_f32";
+  if (!w || !gy || !u || !gu) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (rows == 0 || in_features == 0 || out_features == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
+  OmxGemmEpilogue epi = {OMX_EPI_GELU_BWD, tanh_form ? 1 : 0, u, nullptr};
+  return omx_gemm_impl(ctx, F_LINEAR_BACKWARD, gy, out_features, 1, w, in_features, 1, OMX_F32, gu, OMX_F32, in_features, rows,
+                       out_features, in_features, 0, &epi);
+}
+
 }  // extern "C"

@@ -67,7 +67,7 @@ struct ogpt {
   // Scratch.
   float *e_tok = nullptr, *e_pos = nullptr;
   void *t_a = nullptr, *t_b = nullptr;       // [N,d] AD
-  void *gu = nullptr, *gg = nullptr;         // [N,mlp] AD
+  void* gu = nullptr;                        // [N,mlp] AD
   void *gq = nullptr, *gk = nullptr, *gv = nullptr, *ga = nullptr;  // [N,d] AD
   void* gy16 = nullptr;                      // AD copy of a residual-stream gradient
   // Where the time-major attention takes the head dim: q, k and v are column blocks of one [N, 3d]
@@ -207,8 +207,7 @@ int32_t forward(ogpt* t) {
       // The activation rides in the up-projection's store pass.
       TRY(omx_linear_gelu_forward(ctx, A.h2, t->w(t->li(l, 6)), AD, A.u, A.g, N, d, M, c.gelu_tanh));
     } else {
-      TRY(omx_linear_forward(ctx, A.h2, AD, t->w(t->li(l, 6)), AD, A.u, AD, N, d, M));
-      TRY(omx_gelu_forward(ctx, A.u, A.g, AD, N * M, c.gelu_tanh));
+      TRY(omx_linear_gelu_f32_forward(ctx, A.h2, t->w(t->li(l, 6)), A.u, A.g, N, d, M, c.gelu_tanh));
     }
     TRY(omx_linear_forward(ctx, A.g, AD, t->w(t->li(l, 7)), AD, t->t_a, AD, N, M, d));
     TRY(omx_residual_add_rms_norm_forward(ctx, A.x1, OMX_F32, t->t_a, AD, next_norm, x_next, h_next, AD, N, d, eps));
@@ -256,14 +255,10 @@ int32_t backward(ogpt* t) {
     // Weight gradients go to the arena now, or wait for the batched products after the loop.
     auto gw = [&](uint64_t which) { return defer ? nullptr : t->g(t->li(l, which)); };
     // x_next = x1 + down(gelu(up(norm2(x1))))
-    if (AD == OMX_BF16) {
-      // The activation's derivative rides in the input-gradient product's store pass.
-      if (!defer) TRY(omx_linear_backward(ctx, A.g, nullptr, gy, AD, nullptr, AD, t->g(t->li(l, 7)), OMX_F32, N, M, d));
-      TRY(omx_linear_backward_input_gelu(ctx, t->w(t->li(l, 7)), gy, AD, A.u, gu, N, M, d, c.gelu_tanh));
-    } else {
-      TRY(omx_linear_backward(ctx, A.g, t->w(t->li(l, 7)), gy, AD, t->gg, AD, gw(7), OMX_F32, N, M, d));
-      TRY(omx_gelu_backward(ctx, A.u, t->gg, gu, AD, N * M, c.gelu_tanh));
-    }
+    // The activation's derivative rides in the input-gradient product's store pass.
+    if (!defer) TRY(omx_linear_backward(ctx, A.g, nullptr, gy, AD, nullptr, AD, t->g(t->li(l, 7)), OMX_F32, N, M, d));
+    if (AD == OMX_BF16) TRY(omx_linear_backward_input_gelu(ctx, t->w(t->li(l, 7)), gy, AD, A.u, gu, N, M, d, c.gelu_tanh));
+    else TRY(omx_linear_backward_input_gelu_f32(ctx, t->w(t->li(l, 7)), gy, A.u, gu, N, M, d, c.gelu_tanh));
     TRY(omx_linear_backward(ctx, A.h2, t->w(t->li(l, 6)), gu, AD, t->t_a, AD, gw(6), OMX_F32, N, d, M));
     // Fan-in at x1: the residual branch arrives first, then the norm branch.
     TRY(omx_rms_norm_backward_residual(ctx, A.x1, OMX_F32, t->w32(t->li(l, 5)), t->t_a, AD, gres, gres1, copy_o,
@@ -464,7 +459,6 @@ int32_t create(omx_ctx* ctx, const ogpt_config& c, bool defer, ogpt** out) {
   CREATE_TRY(alloc_act(t, N * d, &t->t_a));
   CREATE_TRY(alloc_act(t, N * d, &t->t_b));
   if (!t->deferred_dw) CREATE_TRY(alloc_act(t, N * M, &t->gu));
-  CREATE_TRY(alloc_act(t, N * M, &t->gg));
   if (t->fused_qkv) {
     if (!t->deferred_dw) CREATE_TRY(alloc_act(t, 3 * N * d, &t->gqkv));
   } else {

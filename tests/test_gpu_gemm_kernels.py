@@ -638,3 +638,27 @@ def test_f32_tiles(be, tile, layout, m, k, n):
                 be.sync()
     finally:
         be.set_option("gemm_f32", -1)
+
+
+@pytest.mark.parametrize("tanh", [0, 1])
+@pytest.mark.parametrize("rows,kin,nout", [(2048, 256, 1024), (70, 288, 36), (65, 256, 61), (513, 1024, 33), (3, 260, 20), (33, 64, 50), (300, 512, 512)])
+def test_f32_activation_in_the_store_pass_carries_the_separate_passes_bits(be, rows, kin, nout, tanh):
+    """`omx_linear_gelu_f32_forward` and `omx_linear_backward_input_gelu_f32` against product and pass: the kernel with the
+    activation in its store pass at the edges of its tiles, and products that it does not take."""
+    from ojas_amd.backend import F32
+
+    print(f"f32 gelu products {rows}x{kin}x{nout} tanh={tanh}", flush=True)
+    be.set_option("gemm_dma", 1)
+    r = np.random.default_rng(rows + kin + nout)
+    x, w, gy = ((r.standard_normal(s) * size).astype(np.float32) for s, size in (((rows, kin), 1.0), ((nout, kin), 0.1), ((rows, kin), 1.0)))
+    dx, dw, u, act = be.upload(x), be.upload(w), be.empty((rows, nout), F32), be.empty((rows, nout), F32)
+    n64 = lambda *v: tuple(C.c_uint64(i) for i in v)
+    p = be._p
+    be._check(be._lib.omx_linear_gelu_f32_forward(be._ctx, p(dx), p(dw), p(u), p(act), *n64(rows, kin, nout), C.c_int32(tanh)))
+    forward, backward = (be.gelu_tanh_forward, be.gelu_tanh_backward) if tanh else (be.gelu_erf_forward, be.gelu_erf_backward)
+    want = be.linear_forward(dx, dw)
+    assert np.array_equal(be.download(u), be.download(want)) and np.array_equal(be.download(act), be.download(forward(want)))
+    # gu [rows, nout] = (gy [rows, kin] . v [kin, nout]) gelu'(u)
+    dv, dg, gu = be.upload(np.ascontiguousarray(w.T)), be.upload(gy), be.empty((rows, nout), F32)
+    be._check(be._lib.omx_linear_backward_input_gelu_f32(be._ctx, p(dv), p(dg), p(u), p(gu), *n64(rows, nout, kin), C.c_int32(tanh)))
+    assert np.array_equal(be.download(gu), be.download(backward(u, be.linear_backward_input(dv, dg))))
