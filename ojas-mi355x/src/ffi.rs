@@ -94,6 +94,8 @@ extern "C" {
     pub fn omx_causal_sdpa_backward_recompute(ctx: *mut OmxCtx, q: *const c_void, k: *const c_void, v: *const c_void, gy: *const c_void, operand_dtype: i32, gy_dtype: i32, gq: *mut c_void, gk: *mut c_void, gv: *mut c_void, grad_dtype: i32, batch: u64, heads: u64, kv_heads: u64, time: u64, head_dim: u64, window: u64) -> i32;
     pub fn omx_linear_gelu_forward(ctx: *mut OmxCtx, x: *const c_void, w: *const c_void, operand_dtype: i32, u: *mut c_void, act: *mut c_void, rows: u64, in_features: u64, out_features: u64, tanh_form: i32) -> i32;
     pub fn omx_linear_backward_input_gelu(ctx: *mut OmxCtx, w: *const c_void, gy: *const c_void, operand_dtype: i32, u: *const c_void, gu: *mut c_void, rows: u64, in_features: u64, out_features: u64, tanh_form: i32) -> i32;
+    pub fn omx_linear_gelu_f32_forward(ctx: *mut OmxCtx, x: *const c_void, w: *const c_void, u: *mut c_void, act: *mut c_void, rows: u64, in_features: u64, out_features: u64, tanh_form: i32) -> i32;
+    pub fn omx_linear_backward_input_gelu_f32(ctx: *mut OmxCtx, w: *const c_void, gy: *const c_void, u: *const c_void, gu: *mut c_void, rows: u64, in_features: u64, out_features: u64, tanh_form: i32) -> i32;
     pub fn omx_causal_attention_forward(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, operand_dtype: i32, out: *mut c_void, out_pitch: u64, out_dtype: i32, lse: *mut c_void, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
     pub fn omx_causal_attention_backward(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, out: *const c_void, gy: *const c_void, out_pitch: u64, lse: *const c_void, operand_dtype: i32, gq: *mut c_void, gk: *mut c_void, gv: *mut c_void, grad_dtype: i32, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
     pub fn omx_causal_attention_forward_saving(ctx: *mut OmxCtx, q: *const c_void, q_pitch: u64, k: *const c_void, v: *const c_void, kv_pitch: u64, operand_dtype: i32, out: *mut c_void, out_residual: *mut c_void, out_pitch: u64, out_dtype: i32, lse: *mut c_void, batch: u64, time: u64, heads: u64, kv_heads: u64, head_dim: u64, window: u64) -> i32;
