@@ -621,7 +621,7 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
   const uint64_t partial_bytes = round_up(blocks * heads * sizeof(float), 256);
   const uint64_t stage_bytes = OMX_COLUMN_SUM_GROUPS * heads * sizeof(float);
   const size_t lds_bytes = static_cast<size_t>(block_rows) * heads * sizeof(float);
-  if (lds_bytes > 64 * 1024) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: %llu heads above 1024", op, (unsigned long long)heads);
+  if (heads > 1024) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: %llu heads above 1024", op, (unsigned long long)heads);  // 64 KiB of LDS
   void* ws = nullptr;
   rc = omx_workspace(ctx, gates_bytes + gz_bytes + partial_bytes + stage_bytes, &ws);
   if (rc != OMX_OK) return rc;

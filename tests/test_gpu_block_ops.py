@@ -661,3 +661,20 @@ def test_elementwise_packs_of_four_and_single(be, n, offset):
     assert np.array_equal(be.download(dy)[offset:], y + x)
     be._check(be._lib.omx_scale_grad(be._ctx, at(dx, 4), C.c_float(0.3), C.c_uint64(n)))
     assert np.array_equal(be.download(dx)[offset:], x * np.float32(0.3))
+
+
+@pytest.mark.parametrize("rows", [8, 4096])
+def test_gate_backward_refuses_more_heads_than_its_widest_block_holds(be, rows):
+    """Whatever the rows per block: 1024 heads are taken, 1025 are not."""
+    from ojas_amd.backend import UNSUPPORTED, OjasError
+
+    for heads, refused in ((1024, False), (1025, True)):
+        x, w, b = be.zeros((rows, 4)), be.zeros((heads, 4)), be.zeros((heads,))
+        attn, gy = be.zeros((rows, heads, 1)), be.zeros((rows, heads, 1))
+        if refused:
+            with pytest.raises(OjasError) as e:
+                be.per_head_sigmoid_gate_backward(x, w, b, attn, gy)
+            assert e.value.code == UNSUPPORTED
+        else:
+            be.per_head_sigmoid_gate_backward(x, w, b, attn, gy)
+            be.sync()
