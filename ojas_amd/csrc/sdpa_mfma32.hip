@@ -34,7 +34,7 @@
 // 23 / 88, 107 / 366.
 //
 // On vector instructions, through shared tiles and now, us, forward / backward (batch x heads over KV heads x time x head
-// dim): 8 x 4/4 x 256 x 64: 38 / 109, 13 / 34, 11 / 30; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370, 20 / 66, 19 / 60; 16 x 12/12
+// dim): 8 x 4/4 x 256 x 64: 38 / 109, 13 / 34, 11 / 30; 2 x 8/2 x 777 x 64 in a window of 256: 47 / 370, 20 / 66, 19 / 55; 16 x 12/12
 // x 512 x 64 (shared tiles still): 272 / 1337, 132 / 439 (48 and 37 TFLOP/s, causal-counted); 16 x 4096 x 64: 587 / 1868 through shared
 // tiles, 325 / 1120; 1 x 2/1 x 3000 x 128: 696 / 3334, 151 / 409, 86 / 216.
 #include <algorithm>
@@ -846,8 +846,12 @@ struct AtGrad {
 };
 
 // dQ, and the row term delta = dO . O when `out` is given (it is read from `delta` otherwise).
+// Three workgroups per compute unit at D = 64, KW = 4: left to itself the compiler takes 172
+// registers, which is two, and 780 workgroups (2 x 8 heads, 777 rows, window 256) leave most of the
+// second of their two rounds idle. At 152, without spills, they fit one: backward 58.8 -> 54.9 us
+// (360 rows, 32 planes 53.3 -> 49.7). At D = 128 a bound of two spills and costs 8-28 %: none there.
 template <int D, int KW>
-__global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
+__global__ __launch_bounds__(AT_THREADS, D == 64 && KW == 4 ? 3 : 1) void sdpa32_dq_kernel(Sdpa32Args a) {
   using X = AtDim<D>;
   constexpr int QW = 4 / KW, BQ = 16 * QW, BLOCKS = KW == 1 ? 4 : 1, KEYS = 16 * BLOCKS;
   __shared__ __align__(16) float lds[KW == 1 ? 2 * AT_ROWS * X::P : 4 * 16 * X::P];
@@ -985,8 +989,10 @@ __global__ __launch_bounds__(AT_THREADS) void sdpa32_dq_kernel(Sdpa32Args a) {
 }
 
 // dK and dV of 16 KG keys, over a share (blockIdx.z of gridDim.z) of the row tiles that see them.
+// Two workgroups per compute unit at D = 128, RW = 1 (LDS allows two; without the bound registers
+// allow one): 512 rows of 64 planes, backward 308 -> 278 us; 12 bytes of a lane go to scratch.
 template <int D, int RW>  // RW waves share a tile's rows, 4 / RW take 16 keys each
-__global__ __launch_bounds__(AT_THREADS) void sdpa32_dkv_kernel(Sdpa32Args a) {
+__global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa32_dkv_kernel(Sdpa32Args a) {
   using X = AtDim<D>;
   // RW = 4: nothing but the waves' sums goes through LDS; row tiles are blocks of 16 rows.
   constexpr int KG = 4 / RW, BK = 16 * KG, NB = AT_ROWS / 16, ROWS = RW == 1 ? AT_ROWS : 16;
