@@ -62,6 +62,7 @@ int32_t omx_fail(omx_ctx* ctx, omx_status code, const char* fmt, ...) {
 // HIP status mapping follows ojas-hip/src/lib.rs:106-122: 2 is out of memory,
 // 3/4/35/100/101 mean no usable device, anything else is a launch failure.
 int32_t omx_hip_fail(omx_ctx* ctx, hipError_t err, const char* what) {
+  (void)hipGetLastError();  // it is reported here: the check after the next launch would find it again
   int code = static_cast<int>(err);
   omx_status st = OMX_BACKEND;
   if (code == 2) st = OMX_CAPACITY_EXCEEDED;
