@@ -94,7 +94,8 @@ int32_t omx_copy(omx_ctx* ctx, void* dst, const void* src, uint64_t bytes);
 int32_t omx_fill_zero(omx_ctx* ctx, void* dst, uint64_t bytes);
 /* Waits for all submitted work; reports and clears a deferred fault. */
 int32_t omx_sync(omx_ctx* ctx);
-/* The context's HIP stream (hipStream_t), for callers that time with events. */
+/* The context's HIP stream (hipStream_t), for callers that time with events or capture graphs. The scratch that a captured op
+ * used stays (charged to the budget) until the context closes; a graph is not to be replayed after that. */
 void* omx_stream(omx_ctx* ctx);
 
 /* ---- casts: BackendCore::{cast_bf16,to_bf16,to_f32} (backend.rs:975-1090),

@@ -298,19 +298,33 @@ int32_t omx_unsupported(omx_ctx* ctx, const char* op) {
 
 namespace {
 uint64_t workspace_size(uint64_t bytes) { return (bytes + (1ull << 20) - 1) & ~((1ull << 20) - 1); }
+
+bool capturing(const omx_ctx* ctx) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
 }  // namespace
 
 bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot) {
   const uint64_t held = ctx->workspace_bytes[slot];
-  return bytes <= held || ctx->budget_limit == 0 || ctx->budget_live - held + workspace_size(bytes) <= ctx->budget_limit;
+  if (bytes <= held || ctx->budget_limit == 0) return true;
+  const uint64_t back = ctx->workspace_captured[slot] || capturing(ctx) ? 0 : held;  // what growing it gives back
+  return ctx->budget_live - back + workspace_size(bytes) <= ctx->budget_limit;
 }
 
 int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot) {
+  const bool in_graph = capturing(ctx);
   if (bytes <= ctx->workspace_bytes[slot]) {
+    ctx->workspace_captured[slot] |= in_graph;
     *out = ctx->workspace[slot];
     return OMX_OK;
   }
-  if (ctx->workspace[slot]) {
+  if (in_graph || ctx->workspace_captured[slot]) {
+    // A captured graph holds the block's address for as long as it is replayed, which nothing tells the context: the block stays,
+    // charged, until the context closes. (In a capture nothing can be waited for, so nothing is freed there either.)
+    ctx->workspace[slot] = nullptr;
+    ctx->workspace_bytes[slot] = 0;
+  } else if (ctx->workspace[slot]) {
     // An outgrown workspace goes back to the driver, not into the pool: its size (a multiple of
     // 1 MiB that only this slot ever asked for) would match no later request and stay parked.
     auto it = ctx->allocations.find(ctx->workspace[slot]);
@@ -327,6 +341,7 @@ int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot) {
   int32_t rc = omx_alloc(ctx, rounded, &ctx->workspace[slot]);
   if (rc != OMX_OK) return rc;
   ctx->workspace_bytes[slot] = rounded;
+  ctx->workspace_captured[slot] = in_graph;
   *out = ctx->workspace[slot];
   return OMX_OK;
 }

@@ -87,6 +87,7 @@ struct omx_ctx {
   // Slot 2: tensors an op keeps across calls into other ops (a recomputed attention output).
   void* workspace[3] = {nullptr, nullptr, nullptr};
   uint64_t workspace_bytes[3] = {0, 0, 0};
+  bool workspace_captured[3] = {false, false, false};  // handed out while the stream was captured
   int cu_count = 0;
   // This device's copy of the static scratch of omx_cross_entropy_mean_forward_static, looked up
   // when the context is opened (the lookup is not stream work and may load the code object).

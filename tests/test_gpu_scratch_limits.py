@@ -1,4 +1,6 @@
 """Ops at the limits of their scratch memory: a full device or budget, and inside a captured graph."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -24,3 +26,54 @@ def test_a_refused_allocation_leaves_the_next_op_alone(be):
         be.empty((1 << 44,))
     assert e.value.code == CAPACITY_EXCEEDED
     assert np.array_equal(be.download(be.residual_add_forward(x, x)), np.full((4, 64), 2.0, np.float32))
+
+
+class Graph:
+    """What `record()` launches on a backend's stream, captured (relaxed, so that it may allocate its results, which it returns)."""
+
+    def __init__(self, be, record):
+        self.hip, self.stream = be._lib, C.c_void_p(be.stream())
+        self.graph, self.program = C.c_void_p(), C.c_void_p()
+        assert self.hip.hipStreamBeginCapture(self.stream, C.c_int(2)) == 0
+        self.results = record()
+        assert self.hip.hipStreamEndCapture(self.stream, C.byref(self.graph)) == 0
+        assert self.hip.hipGraphInstantiate(C.byref(self.program), self.graph, None, None, C.c_size_t(0)) == 0
+
+    def launch(self):
+        assert self.hip.hipGraphLaunch(self.program, self.stream) == 0
+
+    def close(self):
+        self.hip.hipGraphExecDestroy(self.program)
+        self.hip.hipGraphDestroy(self.graph)
+
+
+def load(be, tensor, values):
+    be._check(be._lib.omx_upload(be._ctx, be._p(tensor), C.c_uint64(0), values.ctypes.data_as(C.c_void_p), C.c_uint64(values.nbytes)))
+
+
+def test_a_captured_graph_keeps_the_scratch_it_was_recorded_with():
+    """A later call that needs more takes a block of its own: the graph's stays where it was, and its replays stay right while
+    that call's scratch is written in between."""
+    from ojas_amd.backend import MiBackend
+
+    print("captured argmax, then a norm with more scratch", flush=True)
+    be = MiBackend(0)
+    r = np.random.default_rng(1)
+    x = be.zeros((2, 50257))
+    rows = [be.upload(r.standard_normal((4096, 4096)).astype(np.float32)) for _ in range(2)]
+    w = be.upload(np.ones(4096, np.float32))
+    be.argmax_rows(x)  # grows the workspace: 1 MiB
+    graph = Graph(be, lambda: be.argmax_rows(x))
+    be.sync()
+    live = be.budget()["live"]
+    norm = be.rms_norm_backward(rows[0], w, rows[1])  # 288 rows of partial sums: 5 MiB
+    assert be.budget()["live"] == live + sum(t.nbytes for t in norm) + (5 << 20)
+    want = be.download(norm[1])
+    for _ in range(4):
+        values = r.standard_normal((2, 50257)).astype(np.float32)
+        load(be, x, values)
+        graph.launch()
+        assert np.array_equal(be.download(graph.results), np.argmax(values, axis=1).astype(np.uint32))
+        assert np.array_equal(be.download(be.rms_norm_backward(rows[0], w, rows[1])[1]), want)
+    graph.close()
+    be.close()
