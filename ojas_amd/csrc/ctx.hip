@@ -345,3 +345,9 @@ int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot) {
   *out = ctx->workspace[slot];
   return OMX_OK;
 }
+
+void* omx_workspace_if_room(omx_ctx* ctx, uint64_t bytes, int slot) {
+  if (bytes > ctx->workspace_bytes[slot] && (capturing(ctx) || !omx_workspace_fits(ctx, bytes, slot))) return nullptr;
+  void* ws = nullptr;
+  return omx_workspace(ctx, bytes, &ws, slot) == OMX_OK ? ws : nullptr;
+}

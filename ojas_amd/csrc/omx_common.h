@@ -178,6 +178,9 @@ int32_t omx_hip_fail(omx_ctx* ctx, hipError_t err, const char* what);
 int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot = 0);
 // Whether the budget has room for workspace `slot` at that size (for an op that can do with less).
 bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot = 0);
+// Workspace `slot` for an op that can do without: null where the budget or the device lacks the room, and where a capture would have to
+// allocate it.
+void* omx_workspace_if_room(omx_ctx* ctx, uint64_t bytes, int slot = 0);
 // Next launch tag for fault attribution: (sequence << 8) | op.
 inline unsigned long long omx_tag(omx_ctx* ctx, uint32_t op) {
   return (static_cast<unsigned long long>(++ctx->sequence) << 8) | op;

@@ -985,12 +985,10 @@ int32_t omx_argmax_rows(omx_ctx* ctx, const void* x, uint64_t rows, uint64_t col
                        static_cast<unsigned int>(cols), static_cast<unsigned int*>(out), parts, ctx->fault, omx_tag(ctx, F_ARGMAX));
   };
   // A quarter of a thousand columns feeds a wave; from four thousand on a row has work for sixteen, from sixteen thousand on, where
-  // rows leave compute units empty, for as many workgroups.
-  if (cols >= 16384 && rows * ARGMAX_SLICES <= 256) {
-    void* ws = nullptr;
-    int32_t rc = omx_workspace(ctx, rows * ARGMAX_SLICES * sizeof(uint2), &ws);
-    if (rc != OMX_OK) return rc;
-    parts = static_cast<uint2*>(ws);
+  // rows leave compute units empty, for as many workgroups (without the scratch for their results, one workgroup a row).
+  if (cols >= 16384 && rows * ARGMAX_SLICES <= 256)
+    parts = static_cast<uint2*>(omx_workspace_if_room(ctx, rows * ARGMAX_SLICES * sizeof(uint2)));
+  if (parts) {
     launch(&argmax_rows_kernel<256, ARGMAX_SLICES>, 256, ARGMAX_SLICES);
     OMX_LAUNCH_CHECK(ctx, "argmax_rows_kernel");
     omx_launch(ctx, argmax_meet_kernel, dim3(static_cast<unsigned>(rows)), dim3(64), 0, static_cast<const uint2*>(parts),

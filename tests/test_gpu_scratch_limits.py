@@ -77,3 +77,44 @@ def test_a_captured_graph_keeps_the_scratch_it_was_recorded_with():
         assert np.array_equal(be.download(be.rms_norm_backward(rows[0], w, rows[1])[1]), want)
     graph.close()
     be.close()
+
+
+def with_less(op, arrays, mib):
+    """`op`'s results in a budget that lacks `mib` MiB of what it takes where nothing is scarce."""
+    from ojas_amd.backend import MiBackend
+
+    wide = MiBackend(0)
+    results = op(wide, *[wide.upload(a) for a in arrays])
+    peak = wide.budget()["peak"]
+    del results
+    wide.close()
+    tight = MiBackend(0, budget_bytes=peak - (mib << 20))
+    got = [tight.download(t) for t in op(tight, *[tight.upload(a) for a in arrays])]
+    tight.close()
+    return got
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 16384), (3, 20001), (16, 16384)])
+def test_argmax_without_room_for_scratch(rows, cols):
+    """Under a full budget, and first called in a capture (which takes nothing but the result)."""
+    from ojas_amd.backend import MiBackend
+
+    print(f"argmax {rows}x{cols} without scratch", flush=True)
+    r = np.random.default_rng(cols)
+    draw = lambda: r.integers(-1000, 1000, (rows, cols)).astype(np.float32)  # (ties)
+    values = draw()
+    (got,) = with_less(lambda be, x: (be.argmax_rows(x),), [values], 1)
+    assert np.array_equal(got, np.argmax(values, axis=1).astype(np.uint32))
+    be = MiBackend(0)
+    x = be.upload(values)
+    live = be.budget()["live"]
+    graph = Graph(be, lambda: be.argmax_rows(x))
+    assert be.budget()["live"] == live + graph.results.nbytes
+    for _ in range(3):
+        values = draw()
+        load(be, x, values)
+        graph.launch()
+        want = np.argmax(values, axis=1).astype(np.uint32)
+        assert np.array_equal(be.download(graph.results), want) and np.array_equal(be.download(be.argmax_rows(x)), want)
+    graph.close()
+    be.close()
