@@ -723,9 +723,8 @@ int32_t omx_cached_attention_forward(omx_ctx* ctx, const void* q, const void* k_
     // Few rows over a long cache: their keys are split over workgroups (without the scratch for it, one walks them all).
     m.nparts = omx_sdpa32_key_parts(ctx, m, static_cast<int>(batch), static_cast<int>(head_dim), bf16);
     const uint64_t bytes = rows_total * m.nparts * (head_dim + 2) * sizeof(float);
-    void* ws = nullptr;
-    if (m.nparts > 1 && (!omx_workspace_fits(ctx, bytes) || omx_workspace(ctx, bytes, &ws) != OMX_OK)) m.nparts = 1;
-    m.partial = m.nparts > 1 ? static_cast<float*>(ws) : nullptr;
+    m.partial = m.nparts > 1 ? static_cast<float*>(omx_workspace_if_room(ctx, bytes)) : nullptr;
+    if (!m.partial) m.nparts = 1;
     const int32_t rc = omx_sdpa32_forward(ctx, m, static_cast<int>(batch), static_cast<int>(head_dim), bf16);
     if (rc != OMX_OK || m.nparts == 1) return rc;
     KvArgs merge{};

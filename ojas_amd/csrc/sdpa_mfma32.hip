@@ -1309,12 +1309,9 @@ int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
       if (cost(p) < cost(parts)) parts = p;
   const long total = static_cast<long>(planes) * a.tk * D;
   while (parts > 1 && parts * total * 8 > (256l << 20)) --parts;
-  if (parts > 1) {
-    void* ws = nullptr;
-    int32_t rc = omx_workspace(ctx, static_cast<uint64_t>(parts) * total * 8, &ws, 1);
-    if (rc != OMX_OK) return rc;
-    a.parts = static_cast<float*>(ws);
-  }
+  // (as many as there is room for, down to one workgroup's walk over all rows)
+  for (; parts > 1; --parts)
+    if ((a.parts = static_cast<float*>(omx_workspace_if_room(ctx, static_cast<uint64_t>(parts) * total * 8, 1)))) break;
   dim3 grid(static_cast<unsigned>(blocks), planes, static_cast<unsigned>(parts));
   if (narrow) omx_launch(ctx, (sdpa32_dkv_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
   else omx_launch(ctx, (sdpa32_dkv_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);

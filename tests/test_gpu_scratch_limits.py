@@ -4,6 +4,8 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import oracle_api as orc
+
 pytestmark = pytest.mark.gpu
 
 
@@ -116,5 +118,72 @@ def test_argmax_without_room_for_scratch(rows, cols):
         graph.launch()
         want = np.argmax(values, axis=1).astype(np.uint32)
         assert np.array_equal(be.download(graph.results), want) and np.array_equal(be.download(be.argmax_rows(x)), want)
+    graph.close()
+    be.close()
+
+
+def close(got, want):
+    """Within the f32 tier's 1e-5 of the oracle."""
+    assert np.max(np.abs(got - want)) <= 1e-5 * max(1.0, float(np.max(np.abs(want))))
+
+
+@pytest.mark.parametrize("mib", [1, 2, 4])
+def test_f32_attention_backward_with_room_for_fewer_parts(mib):
+    """Sixteen parts of the rows are 4 MiB of scratch: with room for 3, for 2, for none."""
+    print(f"f32 attention backward, {mib} MiB less", flush=True)
+    r = np.random.default_rng(mib)
+    q, k, v, gy = (r.standard_normal((1, heads, 512, 64)).astype(np.float32) for heads in (4, 1, 1, 4))
+    orc.set_threads(8)
+    out, lse = orc.causal_sdpa_forward(q, k, v)
+    got = with_less(lambda be, *t: be.causal_sdpa_backward(*t), [q, k, v, out, lse, gy], mib)
+    for a, b in zip(got, orc.causal_sdpa_backward(q, k, v, out, lse, gy)):
+        close(a, b)
+
+
+def test_f32_attention_backward_takes_no_scratch_for_parts_inside_a_capture():
+    from ojas_amd.backend import MiBackend
+
+    print("f32 attention backward, captured first", flush=True)
+    r = np.random.default_rng(7)
+    host = [r.standard_normal((1, heads, 512, 64)).astype(np.float32) for heads in (4, 1, 1, 4)]
+    out, lse = orc.causal_sdpa_forward(*host[:3])
+    want = orc.causal_sdpa_backward(*host[:3], out, lse, host[3])
+    be = MiBackend(0)
+    q, k, v, o, l, gy = (be.upload(a) for a in (*host[:3], out, lse, host[3]))
+    small = [be.upload(a[:, :, :16]) for a in (*host[:3], out, lse, host[3])]
+    be.causal_sdpa_backward(*small)  # the row term's scratch, 1 MiB
+    live = be.budget()["live"]
+    graph = Graph(be, lambda: be.causal_sdpa_backward(q, k, v, o, l, gy))
+    assert be.budget()["live"] == live + sum(t.nbytes for t in graph.results)
+    for _ in range(3):
+        for t in graph.results:
+            load(be, t, np.full(t.shape, np.nan, np.float32))
+        graph.launch()
+        for a, b in zip(graph.results, want):
+            close(be.download(a), b)
+        for a, b in zip(be.causal_sdpa_backward(q, k, v, o, l, gy), want):
+            close(be.download(a), b)
+    graph.close()
+    be.close()
+
+
+def test_attention_over_a_long_cache_takes_no_scratch_inside_a_capture():
+    """16 new rows over 4096 positions: the keys' parts are left out where a capture would have to allocate them."""
+    from ojas_amd.backend import MiBackend
+
+    print("cached attention, captured first", flush=True)
+    r = np.random.default_rng(8)
+    q, k, v = (r.standard_normal(s).astype(np.float32) for s in ((1, 16, 2, 64), (1, 4096, 2, 64), (1, 4096, 2, 64)))
+    want = orc.cached_attention_forward(q, k, v, 4096, 0)
+    be = MiBackend(0)
+    held = [be.upload(a) for a in (q, k, v)]
+    live = be.budget()["live"]
+    graph = Graph(be, lambda: be.cached_attention_forward(*held, 4096))
+    assert be.budget()["live"] == live + graph.results.nbytes
+    for _ in range(3):
+        load(be, graph.results, np.full(q.shape, np.nan, np.float32))
+        graph.launch()
+        close(be.download(graph.results), want)
+        close(be.download(be.cached_attention_forward(*held, 4096)), want)
     graph.close()
     be.close()
