@@ -612,14 +612,16 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
     return omx_fail(ctx, OMX_DTYPE, "%s: attn and grad_output must share a dtype", op);
 
   // Workspace: [gates f32][gz in the operand dtype][per-block bias partials][two-stage sum scratch].
-  // 16 rows per block, or 4 where those are under a block per compute unit (1024 rows of 4 x 64: 6.7 us on 64 blocks, 4.3 on 256).
-  const int block_rows = rows < 16ull * 256 ? 4 : 16;
-  const uint64_t blocks = (rows + block_rows - 1) / block_rows;
+  // 16 rows per block, or 4 where those are under a block per compute unit (1024 rows of 4 x 64: 6.7 us on 64 blocks, 4.3 on 256) and
+  // there is room for as many partials.
   const uint64_t items = rows * heads;
   const uint64_t gates_bytes = round_up(items * sizeof(float), 256);
   const uint64_t gz_bytes = round_up(items * omx_dtype_size(operand_dtype), 256);
-  const uint64_t partial_bytes = round_up(blocks * heads * sizeof(float), 256);
   const uint64_t stage_bytes = OMX_COLUMN_SUM_GROUPS * heads * sizeof(float);
+  auto partial_of = [&](uint64_t blocks) { return round_up(blocks * heads * sizeof(float), 256); };
+  const bool few = rows < 16ull * 256 && omx_workspace_fits(ctx, gates_bytes + gz_bytes + partial_of((rows + 3) / 4) + stage_bytes);
+  const int block_rows = few ? 4 : 16;
+  const uint64_t blocks = (rows + block_rows - 1) / block_rows, partial_bytes = partial_of(blocks);
   const size_t lds_bytes = static_cast<size_t>(block_rows) * heads * sizeof(float);
   if (heads > 1024) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: %llu heads above 1024", op, (unsigned long long)heads);  // 64 KiB of LDS
   void* ws = nullptr;

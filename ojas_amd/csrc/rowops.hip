@@ -698,12 +698,14 @@ int32_t launch_rms_fwd(omx_ctx* ctx, const void* x, const float* w, void* y, uin
 template <typename TX, typename TG, typename TO>
 int32_t launch_rms_bwd(omx_ctx* ctx, const void* x, const float* w, const void* gy, void* gx, float* gw,
                        uint64_t rows, uint64_t dim, float eps, unsigned long long tag) {
-  // 32 rows per block, 16 where those are under a block per compute unit, more when that would leave over 2048 partial rows to add.
-  int rows_per_block = rows < 32ull * 256 ? 16 : 32;
+  // 32 rows per block, 16 where those are under a block per compute unit and there is room for as many partial rows, more when that
+  // would leave over 2048 partial rows to add.
+  auto bytes_of = [&](uint64_t blocks) { return (blocks + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float); };
+  int rows_per_block = rows < 32ull * 256 && omx_workspace_fits(ctx, bytes_of((rows + 15) / 16)) ? 16 : 32;
   while ((rows + rows_per_block - 1) / rows_per_block > 2048 && rows_per_block < (1 << 20)) rows_per_block *= 2;
   uint64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
   void* partial = nullptr;
-  int32_t rc = omx_workspace(ctx, (blocks + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float), &partial);
+  int32_t rc = omx_workspace(ctx, bytes_of(blocks), &partial);
   if (rc != OMX_OK) return rc;
   // A narrow row leaves the column sum one or two workgroups: it then adds its rows in two stages.
   float* stage = static_cast<float*>(partial) + blocks * dim;

@@ -187,3 +187,24 @@ def test_attention_over_a_long_cache_takes_no_scratch_inside_a_capture():
         close(be.download(be.cached_attention_forward(*held, 4096)), want)
     graph.close()
     be.close()
+
+
+def test_norm_backward_with_room_for_fewer_partial_rows():
+    """4000 x 2500: 250 partial rows are 3 MiB, 125 are 2."""
+    print("norm backward 4000x2500, 1 MiB less", flush=True)
+    r = np.random.default_rng(1)
+    x, gy = (r.standard_normal((4000, 2500)).astype(np.float32) for _ in range(2))
+    w = (1 + 0.1 * r.standard_normal(2500)).astype(np.float32)
+    for a, b in zip(with_less(lambda be, *t: be.rms_norm_backward(*t), [x, w, gy], 1), orc.rms_norm_backward(x, w, gy)):
+        close(a, b)
+
+
+def test_gate_backward_with_room_for_fewer_partial_rows():
+    """2800 rows of 256 heads: 7 MiB of scratch with 700 partial rows, 6 with 175."""
+    print("gate backward 2800 x 256 heads, 1 MiB less", flush=True)
+    r = np.random.default_rng(2)
+    x, w, b = (0.3 * r.standard_normal(s).astype(np.float32) for s in ((2800, 32), (256, 32), (256,)))
+    attn, gy = (r.standard_normal((2800, 256, 4)).astype(np.float32) for _ in range(2))
+    got = with_less(lambda be, *t: be.per_head_sigmoid_gate_backward(*t), [x, w, b, attn, gy], 1)
+    for a, c in zip(got, orc.gate_backward(x, w, b, attn, gy)):
+        close(a, c)
