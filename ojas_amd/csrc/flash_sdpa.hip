@@ -1194,9 +1194,11 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
   // the chip's workgroup places.
   const unsigned q_blocks = static_cast<unsigned>((s.time + 127) / 128), planes = static_cast<unsigned>(s.batch * s.heads);
   const int tiles = flash_tiles(s);
-  // Head dim 128: from 12 tiles on. Over fewer, two groups gain 0.4 to 4 us (16 heads x 128 / 512: 8.4 -> 8.0, 18.8 -> 14.6), and while
-  // their error against 64 bits is 4 % smaller, the probabilities round elsewhere: the worst adapter gradient of two wide blocks over
-  // 512 tokens went from 0.0185 to 0.0200 of its tensor's largest value, where 0.02 is asked for.
+  // Head dim 128: from 12 tiles on (16 heads x 1024: 32 -> 23 us). A group rounds its probabilities against its own running maximum and not
+  // the row's, which is another rounding of the same width: gradients of adapters against 64 bits keep their error normwise (1.00 of
+  // one group's, 0.99 to 1.01, over 54 models of 512 to 2048 columns and 512 to 2048 positions), while which element is the worst is
+  // chance (two groups / one: 0.81 to 1.28). At 2048 columns it is 0.99 on average from 768 positions on, but 1.03 to 1.10 on each of four
+  // models over 512, so there, where groups gain 0.4 to 4 us (16 heads x 128 / 512: 8.4 -> 8.0, 18.8 -> 14.6), one group stays.
   const int groups = D == 128 && tiles < 12 && ctx->flash_schedule == 0 ? 1 : flash_groups(ctx, planes, s.time, tiles, s.window > 0, D);
   s.q_single = groups > 1 || flash_single(ctx, (q_blocks + 1) / 2 * planes, D == 64 ? 3 : 2, false);
   const unsigned rows = 128 / groups;
@@ -1232,7 +1234,6 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
   // dQ first: it also leaves delta = dO . O per row for the dK/dV pass.
   dim3 block(FT);
   const unsigned pairs = static_cast<unsigned>((s.time + 127) / 128 + 1) / 2;  // two 128-row blocks per workgroup
-  const unsigned blocks = static_cast<unsigned>((s.time + 127) / 128);
   const unsigned kv_planes = static_cast<unsigned>(s.batch * s.kv_heads), q_planes = static_cast<unsigned>(s.batch * s.heads);
   const int tiles = flash_tiles(s);
   const int q_groups = flash_groups(ctx, q_planes, s.time, tiles, s.window > 0, D);

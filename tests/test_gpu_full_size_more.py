@@ -200,6 +200,41 @@ def test_lora_full_width_two_blocks_match_the_oracle(be):
     assert max(normwise) <= 2e-2, normwise
 
 
+@pytest.mark.parametrize("time,seed", [(705, 1), (768, 2), (1100, 3)])
+def test_lora_over_longer_sequences_matches_the_oracle(be, time, seed):
+    """Two blocks of eight heads of 128, where attention's row blocks are shared by groups of waves in the forward too, and
+    without: the bounds of 512 positions."""
+    from ojas_amd.lora import LoraConfig, LoraTrainer
+
+    shape = (2, 1024, 8, 128, 2048, 1000, 1, time, 16)
+    print(f"lora {shape}", flush=True)
+    cfg, ocfg = LoraConfig(*shape, 1e-6, 1.0, 10000.0), orc.LoraConfig(*shape, 1e-6, 1.0, 10000.0)
+    frozen, quant = _frozen_case(ocfg, seed)
+    rng = np.random.default_rng(seed)
+    adapters = [orc.round_bf16(rng.normal(0, 0.02, s).astype(np.float32)) for s in orc.lora_adapter_shapes(ocfg)]
+    ids, targets = (rng.integers(0, ocfg.vocab, time).astype(np.uint32) for _ in range(2))
+    orc.set_threads(16)
+    oloss, ograds = orc.lora_loss_and_grads(ocfg, frozen, adapters, ids, targets)
+    tr = LoraTrainer(be, cfg)
+    try:
+        _load(tr, cfg, frozen, quant)
+        tr.set_adapters(adapters)
+        tr.set_batch(ids, targets)
+        for schedule in (0, 1):  # by the rule: two groups; one
+            be.set_option("flash_schedule", schedule)
+            loss, grads = tr.loss_and_grads(), tr.grads()
+            assert abs(loss - float(oloss)) <= 1e-3 * abs(float(oloss)), (schedule, loss, oloss)
+            elementwise = [float(np.max(np.abs(g - og)) / np.max(np.abs(og))) for g, og in zip(grads, ograds)]
+            normwise = [float(np.linalg.norm(g - og) / np.linalg.norm(og)) for g, og in zip(grads, ograds)]
+            print(f"  schedule {schedule}: worst element / largest {max(elementwise):.4f}, normwise {max(normwise):.4f}", flush=True)
+            # (measured over 12 models of 768 and 1100 positions: at most 1.6e-2 and 1.4e-2 either way)
+            assert max(elementwise) <= 2e-2, elementwise
+            assert max(normwise) <= 2e-2, normwise
+    finally:
+        be.set_option("flash_schedule", 0)
+        tr.close()
+
+
 @pytest.mark.parametrize("kin,nout", [(2048, 6144), (2048, 16384), (8192, 2048)])
 def test_quantised_products_at_full_size_equal_the_bf16_products_of_the_dequantised_weight(be, kin, nout):
     """8192 tokens against the fused q|k|v, gate|up and down matrices of configs[4], in the blocked
