@@ -101,8 +101,8 @@ class NanolabGraph:
         cos, sin = self._rope_tables(T)
         swap = [0, 2, 1, 3]
         # On the backend itself, sums ride in the op that makes their second term (the same bits) and attention reads its
-        # operands as they lie; a wrapper that tags every op's result takes them one by one.
-        fused = isinstance(be, MiBackend)
+        # operands as they lie; a subclass or wrapper, which may count, tag or check single ops, takes them one by one.
+        fused = type(be) is MiBackend
         time_major = fused and D in (16, 32, 64, 128)
 
         def add_norm(x, y, w):

@@ -257,3 +257,41 @@ def test_save_then_resume_continues_bit_for_bit(be, tmp_path):
             resume_checkpoint(be, ckpt, TrainConfig(**{**cfg.__dict__, **other}), tokenizer_hash=bytes(range(32)))
     with pytest.raises(IoError, match="tokenizer hash"):
         resume_checkpoint(be, ckpt, cfg)
+
+
+def test_a_subclass_sees_every_op(be):
+    """A backend whose ops are overridden gets them one by one, as a wrapper does; the backend itself fuses some, with the same results."""
+    from ojas_amd.backend import MiBackend
+    from ojas_amd.nanolab import NanolabSpec
+
+    seen = {}
+
+    class Counting(MiBackend):
+        pass
+
+    def counted(name):
+        def op(self, *args, **kwargs):
+            seen[name] = seen.get(name, 0) + 1
+            return getattr(MiBackend, name)(self, *args, **kwargs)
+
+        return op
+
+    ops = ("residual_add_forward", "permute", "rms_norm_forward", "rms_norm_backward", "causal_sdpa_forward", "causal_sdpa_backward")
+    for name in ops:
+        setattr(Counting, name, counted(name))
+    print("nanolab graph on a subclass", flush=True)
+    spec = NanolabSpec(n_layer=2, n_embd=64, n_head=2, n_kv_head=1, head_dim=32, hidden=96, vocab=64, window=None, max_seq=16)
+    r = np.random.default_rng(0)
+    host = {n: (r.standard_normal(s) * 0.1 if len(s) == 2 else np.ones(s)).astype(np.float32) for n, s in spec.param_shapes().items()}
+    ids, targets = (r.integers(0, 64, (1, 16)).astype(np.uint32) for _ in range(2))
+    sub = Counting(0)
+    loss, _, grads = run(sub, spec, host, ids, targets)
+    # A layer: six sums at least; q, k, v and the output permuted each way; two norms, and the last one.
+    assert seen["residual_add_forward"] >= 2 * 6 and seen["permute"] == 2 * 8, seen
+    assert seen["rms_norm_forward"] == seen["rms_norm_backward"] == 5, seen
+    assert seen["causal_sdpa_forward"] == seen["causal_sdpa_backward"] == 2, seen
+    plain_loss, _, plain = run(be, spec, host, ids, targets)
+    assert abs(loss - plain_loss) <= FORWARD_LOSS_REL_TOL * abs(plain_loss)
+    for name, g in grads.items():
+        assert np.linalg.norm(g - plain[name]) <= GRAD_NORMWISE_REL_TOL * max(np.linalg.norm(plain[name]), 1e-12), name
+    sub.close()
