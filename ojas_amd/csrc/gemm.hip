@@ -834,6 +834,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   }
   g.fault = ctx->fault;
   g.tag = omx_tag(ctx, fault_op);
+  g.act_tag = act_fused ? omx_tag(ctx, act32->mode == OMX_EPI_GELU_FWD ? F_GELU_FORWARD : F_GELU_BACKWARD) : g.tag;
   omx_ctx::TimedLaunch timed{};
   if (ctx->profile_gemm) {
     auto take = [&](hipEvent_t* e) -> hipError_t {

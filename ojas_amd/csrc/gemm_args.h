@@ -22,7 +22,7 @@ struct GemmArgs {
   unsigned short* aux_out;
   float epi_s1, epi_s2;  // OMX_EPI_AXPBY
   OmxFaultWord* fault;
-  unsigned long long tag;
+  unsigned long long tag, act_tag;  // act_tag: of the f32 store pass's activation
   // Strided batch: block (x, y) works on product y, whose operands start batch_* BYTES after
   // product y - 1's. batches == 1 for a single product.
   int batches;
@@ -38,7 +38,7 @@ __device__ __forceinline__ void gemm_select_batch(GemmArgs& g, int product) {
     g.c = static_cast<char*>(g.c) + y * g.batch_c;
     // A split product of a batch keeps its partial sums behind the earlier products'.
     if (g.splits > 1) g.partial += y * g.splits * static_cast<long>(g.M) * g.N;
-    // aux tensors are bf16 like the output they accompany: the same byte stride.
+    // aux tensors have the output's type and layout (f32 with a two-term sum, bf16 with the rest): the same byte stride.
     if (g.aux_in) g.aux_in = reinterpret_cast<const unsigned short*>(reinterpret_cast<const char*>(g.aux_in) + y * g.batch_c);
     if (g.aux_out) g.aux_out = reinterpret_cast<unsigned short*>(reinterpret_cast<char*>(g.aux_out) + y * g.batch_c);
   }
@@ -107,25 +107,26 @@ __device__ __forceinline__ bool gemm_store4(const GemmArgs& g, int split, int gr
 }
 
 // The f32 product with its activation: C = the value and aux_out = GELU of it, or C = the value times GELU' of aux_in (f32 all, C's
-// layout), as a pass of its own over the stored product would form them.
+// layout), as a pass of its own over the stored product would form them. Returns which is not finite: 1 the product, 2 the activation.
 template <bool TANH>
-__device__ __forceinline__ bool gemm_store4_act32(const GemmArgs& g, int grow, int gcol, float x0, float x1, float x2, float x3) {
+__device__ __forceinline__ int gemm_store4_act32(const GemmArgs& g, int grow, int gcol, float x0, float x1, float x2, float x3) {
   const long off = static_cast<long>(grow) * g.ldc + gcol;
   float x[4] = {x0, x1, x2, x3};
   const int n = min(4, g.N - gcol);
   const bool whole = g.c_vec != 0 && n == 4;
-  bool bad = false;
+  int bad = 0;
   if (g.epi == OMX_EPI_GELU_FWD) {
     float y[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       y[e] = dev_gelu_of<float, TANH>(x[e]);
-      if (e < n) bad |= !dev_finite(y[e]);
+      if (e < n && !dev_finite(y[e])) bad |= 2;
     }
     float* to = reinterpret_cast<float*>(g.aux_out) + off;
     if (whole) *reinterpret_cast<float4*>(to) = make_float4(y[0], y[1], y[2], y[3]);
     else
       for (int e = 0; e < n; ++e) to[e] = y[e];
+    if (gemm_store4(g, 0, grow, gcol, x[0], x[1], x[2], x[3])) bad |= 1;
   } else {
     const float* u = reinterpret_cast<const float*>(g.aux_in) + off;
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -133,9 +134,13 @@ __device__ __forceinline__ bool gemm_store4_act32(const GemmArgs& g, int grow, i
     else
       for (int e = 0; e < n; ++e) v[e] = u[e];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = x[e] * dev_gelu_grad_of<float, TANH>(v[e]);
+    for (int e = 0; e < 4; ++e) {
+      if (e < n && !dev_finite(x[e])) bad |= 1;
+      x[e] = x[e] * dev_gelu_grad_of<float, TANH>(v[e]);
+    }
+    if (gemm_store4(g, 0, grow, gcol, x[0], x[1], x[2], x[3])) bad |= 2;
   }
-  return gemm_store4(g, 0, grow, gcol, x[0], x[1], x[2], x[3]) || bad;
+  return bad;
 }
 
 // gemm_store4 with the optional activation of OmxGemmEpilogue applied first (bf16 outputs, no

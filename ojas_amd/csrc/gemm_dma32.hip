@@ -208,7 +208,7 @@ gemm_dma32_kernel(GemmArgs g) {
   }
   // acc[m][n][v]: A's row i = lane % 16 of block m, B's row 4 (lane / 16) + v of block n.
   const int i = lane & 15, kg = lane >> 4;
-  bool bad = false;
+  int bad = 0;
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
     const int row = m0 + wm * TM * 16 + (A_KM ? TM * i + m : 16 * m + i);
@@ -229,7 +229,8 @@ gemm_dma32_kernel(GemmArgs g) {
       }
     }
   }
-  if (bad) dev_raise_fault(g.fault, g.tag);
+  if (bad & 1) dev_raise_fault(g.fault, g.tag);
+  if (ACT != 0 && (bad & 2)) dev_raise_fault(g.fault, g.act_tag);
 }
 
 template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int NST, int KG>

@@ -662,3 +662,44 @@ def test_f32_activation_in_the_store_pass_carries_the_separate_passes_bits(be, r
     dv, dg, gu = be.upload(np.ascontiguousarray(w.T)), be.upload(gy), be.empty((rows, nout), F32)
     be._check(be._lib.omx_linear_backward_input_gelu_f32(be._ctx, p(dv), p(dg), p(u), p(gu), *n64(rows, nout, kin), C.c_int32(tanh)))
     assert np.array_equal(be.download(gu), be.download(backward(u, be.linear_backward_input(dv, dg))))
+
+
+@pytest.mark.parametrize("tile", [5, 6, 7, 8, 9])  # gemm_dma32.hip's, whose store pass forms the activation; the kernel before a pass of its own
+@pytest.mark.parametrize("tanh", [0, 1])
+def test_f32_activation_in_the_store_pass_is_named_as_the_separate_pass_is(be, tile, tanh):
+    """A product that is not finite carries the product's name, an activation that is not the activation's."""
+    from ojas_amd.backend import OjasError
+
+    print(f"f32 gelu products, fault names, tile {tile} tanh={tanh}", flush=True)
+    r = np.random.default_rng(tile)
+    rows, nin, nout = 70, 260, 256
+    n64 = lambda *v: tuple(C.c_uint64(i) for i in v)
+    p = be._p
+
+    def backward(gy, w, u):
+        gu = be.empty(u.shape)
+        be._check(be._lib.omx_linear_backward_input_gelu_f32(be._ctx, p(w), p(gy), p(u), p(gu), *n64(rows, nin, nout), C.c_int32(tanh)))
+
+    def forward(x, w):
+        u, act = be.empty((rows, nin)), be.empty((rows, nin))
+        be._check(be._lib.omx_linear_gelu_f32_forward(be._ctx, p(x), p(w), p(u), p(act), *n64(rows, nout, nin), C.c_int32(tanh)))
+
+    w, gy, u = (r.standard_normal(s).astype(np.float32) for s in ((nout, nin), (rows, nout), (rows, nin)))
+    bad_gy, bad_u, huge_gy, huge_w, peak_u = gy.copy(), u.copy(), np.zeros_like(gy), np.zeros_like(w), u.copy()
+    bad_gy[-1, 4] = np.inf
+    bad_u[69, 259] = np.nan
+    huge_gy[3, 0], huge_w[0, 5], peak_u[3, 5] = 3.2e38, 1.0, 1.4  # a finite product, 1.13 times too large
+    cases = [(backward, (bad_gy, w, u), "linear_backward"), (backward, (gy, w, bad_u), "gelu_backward"),
+             (backward, (huge_gy, huge_w, peak_u), "gelu_backward"), (forward, (bad_gy, np.ascontiguousarray(w.T)), "linear_forward")]
+    be.set_option("gemm_dma", 1)
+    be.set_option("gemm_f32", tile)
+    try:
+        for op, args, name in cases:
+            op(*[be.upload(a) for a in args])
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.detail == name, (tile, e.value.detail)
+        backward(*[be.upload(a) for a in (gy, w, u)])
+        be.sync()
+    finally:
+        be.set_option("gemm_f32", -1)
