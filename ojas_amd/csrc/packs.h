@@ -1,6 +1,7 @@
 // Elementwise passes over packs: how many a thread takes, and how it reads and writes one.
 #pragma once
 
+#include <algorithm>
 #include <initializer_list>
 
 #include "omx_common.h"
@@ -8,7 +9,7 @@
 namespace {
 
 constexpr int BK_THREADS = 256;
-constexpr int BK_PACKS = 4;  // packs per thread at most
+constexpr int BK_PACKS = 4;  // packs per thread of a large pass
 
 // A pack is V consecutive elements: one 16-byte (f32) or 8-byte (bf16) access
 // when V == 4, one element when V == 1.
@@ -39,14 +40,20 @@ __device__ __forceinline__ void store_pack(T* __restrict__ p, size_t pack, const
   }
 }
 
-// Packs per thread: one up to four blocks per compute unit, two up to eight, BK_PACKS beyond. A few thousand rows were 16 to 176
+// Packs per thread: one up to four blocks per compute unit, two up to eight, four beyond (and twice that as often as it takes to keep a
+// launch under the 2^32 threads it may have). A few thousand rows were 16 to 176
 // blocks whose threads took their packs one latency after the other (rope over 1024 x 4 x 64 6.3 us on 32 blocks, 3.2 on 128).
+// `blocks`: the most there may be, or (in a kernel) how many there are, which gives the same answer.
 __host__ __device__ inline uint64_t packs_per_thread(uint64_t packs, uint64_t blocks) {
-  return packs <= blocks * BK_THREADS ? 1 : packs <= blocks * (2 * BK_THREADS) ? 2 : BK_PACKS;
+  if (packs <= blocks * BK_THREADS) return 1;
+  uint64_t each = 2;
+  while (packs > blocks * (each * BK_THREADS)) each *= 2;
+  return each;
 }
 inline dim3 pack_grid(uint64_t packs) {
-  const uint64_t each = packs_per_thread(packs, 1024), per_block = each * BK_THREADS;
-  const uint64_t blocks = (packs + per_block - 1) / per_block;
+  constexpr uint64_t FEW = 1024, MOST = (1ull << 32) / BK_THREADS - 1;
+  const uint64_t each = packs <= FEW * (2 * BK_THREADS) ? packs_per_thread(packs, FEW) : std::max<uint64_t>(BK_PACKS, packs_per_thread(packs, MOST));
+  const uint64_t per_block = each * BK_THREADS, blocks = (packs + per_block - 1) / per_block;
   return dim3(static_cast<unsigned>(blocks > 0 ? blocks : 1));
 }
 #define PACK_LOOP(p, packs)                                                                                             \

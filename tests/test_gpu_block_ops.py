@@ -678,3 +678,27 @@ def test_gate_backward_refuses_more_heads_than_its_widest_block_holds(be, rows):
         else:
             be.per_head_sigmoid_gate_backward(x, w, b, attn, gy)
             be.sync()
+
+
+def test_a_pass_of_more_elements_than_four_to_a_thread_allows(be):
+    """2^34 + 1 elements, which cannot be taken in packs of four: a fill and a scaling in place (64 GiB)."""
+    n = (1 << 34) + 1
+    print("fill and scale 64 GiB", flush=True)
+    t = be.zeros((n,))
+    three = np.array([1.0, 2.0, 3.0], np.float32)
+    places = (0, n // 2, n - 3)
+    at = lambda i: C.c_uint64(4 * i)
+
+    def read(i):
+        out = np.empty(3, np.float32)
+        be._check(be._lib.omx_download(be._ctx, out.ctypes.data_as(C.c_void_p), be._p(t), at(i), at(3)))
+        return out
+
+    for i in places:
+        be._check(be._lib.omx_upload(be._ctx, be._p(t), at(i), three.ctypes.data_as(C.c_void_p), at(3)))
+    be.scale_grad(t, 2.0)
+    for i in places:
+        assert np.array_equal(read(i), 2 * three), i
+    be._check(be._lib.omx_fill_zero(be._ctx, be._p(t), at(n)))
+    for i in places:
+        assert not read(i).any(), i
