@@ -118,14 +118,22 @@ struct omx_ctx {
   };
   std::vector<TimedLaunch> timed;
   std::vector<hipEvent_t> event_pool;
+  bool launch_too_large = false;  // since the last OMX_LAUNCH_CHECK
 };
 
 // A kernel launch on the context's stream, the arguments converted to the kernel's parameter types. Straight through
 // hipLaunchKernel: the <<<>>> form pushes the launch's shape onto a stack and pops it again in a stub of the kernel's,
 // 0.25 us more of host time (3.1 -> 2.8 us), which is what bounds a chain of small kernels.
+// A launch has at most 2^32 threads along an axis. The runtime multiplies in 32 bits and runs what is left of a larger one.
+inline bool omx_launchable(omx_ctx* ctx, dim3 grid, dim3 block) {
+  const bool fits = static_cast<uint64_t>(grid.x) * block.x <= 0xffffffffull && static_cast<uint64_t>(grid.y) * block.y <= 0xffffffffull;
+  ctx->launch_too_large |= !fits;
+  return fits;
+}
 template <typename... P, typename... Args>
 inline void omx_launch(omx_ctx* ctx, void (*kernel)(P...), dim3 grid, dim3 block, unsigned smem, Args... args) {
   static_assert(sizeof...(P) == sizeof...(Args), "one argument for each parameter");
+  if (!omx_launchable(ctx, grid, block)) return;
   std::tuple<P...> packed(static_cast<P>(args)...);
   void* at[sizeof...(P) ? sizeof...(P) : 1];
   std::apply([&](auto&... a) {
@@ -139,6 +147,7 @@ inline void omx_launch(omx_ctx* ctx, void (*kernel)(P...), dim3 grid, dim3 block
 template <typename F, typename... Args>
 inline void omx_launch_timed(omx_ctx* ctx, F kernel, dim3 grid, dim3 block, unsigned smem, hipEvent_t start,
                              hipEvent_t stop, Args... args) {
+  if ((start || stop) && !omx_launchable(ctx, grid, block)) return;
   if (start || stop) hipExtLaunchKernelGGL(kernel, grid, block, smem, ctx->stream, start, stop, 0, args...);
   else omx_launch(ctx, kernel, grid, block, smem, args...);
 }
@@ -240,6 +249,10 @@ int32_t omx_convert(omx_ctx* ctx, const void* src, int32_t src_dtype, void* dst,
   do {                                                            \
     hipError_t e_ = hipGetLastError();                            \
     if (e_ != hipSuccess) return omx_hip_fail(ctx, e_, what);     \
+    if ((ctx)->launch_too_large) {                                \
+      (ctx)->launch_too_large = false;                            \
+      return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: more threads than a launch may have", what); \
+    }                                                             \
   } while (0)
 
 #define OMX_REQUIRE_CTX(ctx) \

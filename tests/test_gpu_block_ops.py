@@ -702,3 +702,15 @@ def test_a_pass_of_more_elements_than_four_to_a_thread_allows(be):
     be._check(be._lib.omx_fill_zero(be._ctx, be._p(t), at(n)))
     for i in places:
         assert not read(i).any(), i
+
+
+def test_a_launch_of_more_threads_than_there_may_be_is_refused(be):
+    """2^26 + 8 rows of a wave each are 2^32 + 512 threads, of which the runtime would run 512; the next op is not touched."""
+    from ojas_amd.backend import OUT_OF_RANGE, OjasError
+
+    print("embedding of 2^26 + 8 tokens", flush=True)
+    table, ids = be.upload(np.ones((2, 1), np.float32)), be.upload(np.zeros((1 << 26) + 8, np.uint32))
+    with pytest.raises(OjasError) as e:
+        be.embedding_forward(table, ids)
+    assert e.value.code == OUT_OF_RANGE
+    assert np.array_equal(be.download(be.residual_add_forward(table, table)), np.full((2, 1), 2.0, np.float32))
