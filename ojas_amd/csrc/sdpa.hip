@@ -114,6 +114,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_fwd_rows_kernel(const TI* __r
         acc[i] = a;
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
   bad |= !(dev_finite(run_sum) && run_sum > 0.0f);
@@ -222,6 +223,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dq_rows_kernel(
         acc[i] = a;
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
 #pragma unroll
@@ -305,6 +307,7 @@ __global__ __launch_bounds__(SD_THREADS) void sdpa_bwd_dkv_rows_kernel(
           accv[i] = av;
         }
       }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       __builtin_amdgcn_wave_barrier();
     }
   }

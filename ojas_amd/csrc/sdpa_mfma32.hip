@@ -949,8 +949,10 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && KW == 4 ? 3 : 1) void sdpa32
       values[set].fetch(at_bytes(vb + key0 * a.k_t), off);
     };
     auto step = [&](int set, int t) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();  // the previous block has been read
       at_stage<D>(keys[set], own, i, g);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
       fetch(set ^ 1, min(t + KW, t_last));
       const floatx4_a s = keys[set].dot(q), dp = values[set].dot(dout);
@@ -1123,9 +1125,11 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
       }
     };
     auto step = [&](int set, int u_now) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();  // the previous block has been read
       at_stage<D>(qn[set], own_q, i, g);
       at_stage<D>(gn[set], own_g, i, g);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
       if constexpr (SETS == 2) fetch(set ^ 1, min(u_now + RW, u1 - 1));
       const floatx4_a s = qn[set].dot(k), dp = gn[set].dot(v4);
