@@ -824,7 +824,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     if (!aligned16(sum32->aux_in)) g.c_vec = 0;
   }
   if (epi && !((!epi->aux_in || aligned16(epi->aux_in)) && (!epi->aux_out || aligned16(epi->aux_out)))) g.c_vec = 0;
-  const bool act_fused = act32 && dma32 >= 0 && !a_km && g.splits == 1;
+  const bool act_fused = act32 && dma32 >= 0 && !a_km;  // (never split)
   if (act_fused) {
     g.epi = act32->mode;
     g.epi_tanh = act32->tanh_form;

@@ -83,17 +83,7 @@ gemm_dma32_kernel(GemmArgs g) {
   constexpr int LPS = STAGE / 1024 / NW;  // loads per wave per step
   static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0, "the same number of loads in every wave");
   const int total = g.tiles_m * g.tiles_n;
-  int split = 0, id = blockIdx.x, product = 0;
-  if (g.splits > 1) {
-    split = blockIdx.x % g.splits;
-    id = blockIdx.x / g.splits;
-    product = id / total;
-    id -= product * total;
-  } else {
-    const int r = tile_of_eighth(blockIdx.x, total * g.batches);
-    product = r / total;
-    id = r - product * total;
-  }
+  const int r = tile_of_eighth(blockIdx.x, total * g.batches), product = r / total, id = r - product * total;
   const int band = 4, band_id = id / (band * g.tiles_n), first_m = band_id * band;
   const int band_rows = min(band, g.tiles_m - first_m), in_band = id - band_id * (band * g.tiles_n);
   const int m0 = (first_m + in_band % band_rows) * BM, n0 = in_band / band_rows * BN;
@@ -108,14 +98,14 @@ gemm_dma32_kernel(GemmArgs g) {
 #pragma unroll
     for (int n = 0; n < TN; ++n) acc[m][n] = sum[m][n] = floatx4_d{0.0f, 0.0f, 0.0f, 0.0f};
 
-  const int first = split * g.ksteps_per_split, last = min(g.K / BK, first + g.ksteps_per_split);
-  const int rounds = (last - first + KG - 1) / KG;  // of every group
-  const int mine = (last - first - group + KG - 1) / KG;
+  const int steps = g.K / BK;
+  const int rounds = (steps + KG - 1) / KG;  // of every group
+  const int mine = (steps - group + KG - 1) / KG;
   // (an f32 tile's pieces are those of a bf16 one with twice the columns)
   constexpr int KIND = A_KM && B_KM ? 1 : 2;
   TileLoadsOff<A_KM, A_KM ? 2 * BM : BM, A_KM ? BK : 2 * BK, NW, TAIL && A_KM, KIND> la;
   TileLoadsOff<B_KM, B_KM ? 2 * BN : BN, B_KM ? BK : 2 * BK, NW, TAIL && B_KM, KIND> lb;
-  const int k0 = (first + group) * BK;
+  const int k0 = group * BK;
   la.init(static_cast<const unsigned short*>(g.a), 2 * g.lda, A_KM ? 2 * m0 : m0, A_KM ? 2 * g.M : g.M, A_KM ? k0 : 2 * k0, g.k_rows, wave, lane);
   lb.init(static_cast<const unsigned short*>(g.b), 2 * g.ldb, B_KM ? 2 * n0 : n0, B_KM ? 2 * g.N : g.N, B_KM ? k0 : 2 * k0, g.k_rows, wave, lane);
   Frag32Lds<A_KM, BM, TM, KIND> fa;
@@ -223,7 +213,7 @@ gemm_dma32_kernel(GemmArgs g) {
           else x[e] = acc[m][p][e];
         }
         if (col < g.N) {
-          if constexpr (ACT == 0) bad |= gemm_store4(g, split, row, col, x[0], x[1], x[2], x[3]);
+          if constexpr (ACT == 0) bad |= gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3]);
           else bad |= gemm_store4_act32<ACT == 2>(g, row, col, x[0], x[1], x[2], x[3]);
         }
       }
@@ -246,8 +236,8 @@ int32_t launch_dma32(omx_ctx* ctx, const GemmArgs& g) {
   }
   if constexpr (smem > 64 * 1024)
     OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-  omx_launch_timed(ctx, kernel, dim3(static_cast<unsigned>(g.tiles_m) * g.tiles_n * g.batches * g.splits), dim3(WGM * WGN * KG * 64), smem,
-                   ctx->timing_start, g.splits > 1 ? nullptr : ctx->timing_stop, g);
+  omx_launch_timed(ctx, kernel, dim3(static_cast<unsigned>(g.tiles_m) * g.tiles_n * g.batches), dim3(WGM * WGN * KG * 64), smem,
+                   ctx->timing_start, ctx->timing_stop, g);
   OMX_LAUNCH_CHECK(ctx, "gemm_dma32_kernel");
   return OMX_OK;
 }

@@ -1270,14 +1270,10 @@ int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) 
     }
   }
   const bool narrow = per == 16;
-  using Cache = std::conditional_t<(D < 64), unsigned short, float>;  // bf16 caches of wider heads: prompt or (past 32 bits) wide
-  if (narrow) {
-    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, Cache>), grid, dim3(AT_THREADS), 0, a);
-    else omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, float>), grid, dim3(AT_THREADS), 0, a);
-  } else {
-    if (bf16_cache) omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, unsigned short>), grid, dim3(AT_THREADS), 0, a);
-    else omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, float>), grid, dim3(AT_THREADS), 0, a);
-  }
+  if (!bf16_cache) omx_launch(ctx, (narrow ? &sdpa32_fwd_kernel<D, 4, float> : &sdpa32_fwd_kernel<D, 1, float>), grid, dim3(AT_THREADS), 0, a);
+  else if (!narrow) omx_launch(ctx, (sdpa32_fwd_kernel<D, 1, unsigned short>), grid, dim3(AT_THREADS), 0, a);
+  else if constexpr (D < 64) omx_launch(ctx, (sdpa32_fwd_kernel<D, 4, unsigned short>), grid, dim3(AT_THREADS), 0, a);
+  else return omx_fail(ctx, OMX_UNSUPPORTED, "cached attention: no narrow form over bf16 caches of head_dim %d", D);  // (prompt or wide)
   OMX_LAUNCH_CHECK(ctx, "sdpa32_fwd_kernel");
   return OMX_OK;
 }
