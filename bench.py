@@ -53,7 +53,7 @@ KERNEL_CLASSES = [
     (4, "adamw", "adamw_apply_kernel (after adamw_check_kernel when it runs)", "hbm"),
     (5, "rms_norm_forward", "rms_fwd_vec_kernel", "hbm"),
     (6, "rms_norm_backward", "rms_bwd_vec_kernel + column_sum kernels", "hbm"),
-    (7, "embedding_backward", "count / scan / fill / sort kernels + embedding_bwd_kernel", "hbm"),
+    (7, "embedding_backward", "index_ids_kernel, or count / scan / fill kernels, + embedding_bwd_kernel", "hbm"),
 ]
 ALL_CLASSES_MASK = 0xFF
 

@@ -17,8 +17,8 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   int splits, ksteps_per_split;  // split-K: each split writes an f32 partial
   float* partial;                // [splits][M][N] when splits > 1
-  int epi, epi_tanh;             // OMX_EPI_* (bf16 output, no split)
-  const unsigned short* aux_in;
+  int epi, epi_tanh;             // OMX_EPI_* (no split)
+  const unsigned short* aux_in;  // of the output's type: f32 in disguise where that is
   unsigned short* aux_out;
   float epi_s1, epi_s2;  // OMX_EPI_AXPBY
   OmxFaultWord* fault;

@@ -196,9 +196,10 @@ inline unsigned long long omx_tag(omx_ctx* ctx, uint32_t op) {
 }
 
 // C[m,n] (+)= A.B with element strides; `ldc` is C's row pitch in elements.
-// Optional elementwise work in the GEMM's store pass (bf16 outputs only; `aux` shares C's row pitch):
-//   OMX_EPI_GELU_FWD: C = u (rounded to bf16) and aux_out = gelu(u);
-//   OMX_EPI_GELU_BWD: C = round_bf16(A.B) * gelu'(aux_in);
+// Optional elementwise work in the GEMM's store pass (bf16 outputs, or f32 throughout; `aux` has C's type and row pitch):
+//   OMX_EPI_GELU_FWD: C = u (rounded to bf16) and aux_out = gelu(u). f32: nothing is rounded between, and shapes without a store pass
+//     for it take a pass of its own;
+//   OMX_EPI_GELU_BWD: C = round_bf16(A.B) * gelu'(aux_in). f32: as above;
 //   OMX_EPI_AXPBY: C = round_bf16(s1 aux_in) + round_bf16(s2 round_bf16(A.B)): the product stored as
 //     bf16, then the two-term sum a separate pass over it would form, in one store. f32 operands and output: C = s1 aux_in +
 //     s2 A.B, each term rounded as a pass of its own would.
