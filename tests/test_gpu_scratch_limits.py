@@ -81,6 +81,32 @@ def test_a_captured_graph_keeps_the_scratch_it_was_recorded_with():
     be.close()
 
 
+def test_scratch_that_grows_inside_a_capture_leaves_the_smaller_block():
+    """An op that cannot do without: the capture ends well, the block from before it stays, and so does the new one after it."""
+    from ojas_amd.backend import MiBackend
+
+    print("norm backward captured over a smaller workspace", flush=True)
+    be = MiBackend(0)
+    r = np.random.default_rng(3)
+    x, gy = (r.standard_normal((4096, 4096)).astype(np.float32) for _ in range(2))
+    w = np.ones(4096, np.float32)
+    held = [be.upload(a) for a in (x, w, gy)]
+    be.argmax_rows(be.zeros((1, 20000)))  # 1 MiB
+    live = be.budget()["live"]
+    graph = Graph(be, lambda: be.rms_norm_backward(*held))
+    assert be.budget()["live"] == live + sum(t.nbytes for t in graph.results) + (5 << 20)
+    want = orc.rms_norm_backward(x, w, gy)
+    for _ in range(3):
+        for t in graph.results:
+            load(be, t, np.full(t.shape, np.nan, np.float32))
+        graph.launch()
+        for a, b in zip(graph.results, want):
+            assert np.max(np.abs(be.download(a) - b)) <= 1e-5 * max(1.0, float(np.max(np.abs(b))))
+        be.argmax_rows(be.zeros((1, 20000)))
+    graph.close()
+    be.close()
+
+
 def with_less(op, arrays, mib):
     """`op`'s results in a budget that lacks `mib` MiB of what it takes where nothing is scarce."""
     from ojas_amd.backend import MiBackend
