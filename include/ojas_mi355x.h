@@ -151,8 +151,9 @@ int32_t omx_gemm_pitched_strided_batch(omx_ctx* ctx, const void* a, uint64_t a_r
 /* A frozen linear layer whose weight is stored as symmetric int8 codes [n_out, k_in] with one f32
  * scale per `group` consecutive input columns [n_out, k_in / group] (value = code * scale: the
  * per-channel form of ojas-cpu/src/quant_sparse.rs:284-346 applied to groups; group must be 32).
- * The codes are widened inside the product, on their way from HBM to the matrix units; no bf16
- * copy of the weight exists in memory. In the reference a quantised base reaches the graph as
+ * The codes are widened inside the product, on their way from HBM to the matrix units, or, where that is
+ * ahead and the budget has room, into scratch that the next product writes over (at most 1 GiB, given back to any
+ * allocation that would be refused; the same bits either way). No bf16 copy of a weight is kept. In the reference a quantised base reaches the graph as
  * dequantise -> linear_forward (ojas-autograd/src/tape.rs:1514-1518, backend.rs:2586); these two
  * entry points serve that pair of calls for a frozen base, forward and input gradient (a frozen
  * weight has no gradient, ojas-model/src/lora.rs:4-8).
@@ -677,7 +678,8 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * two wave groups / 32 x 32 by four, wherever the operands fit it, 9 = the register-staged kernel.
  * "gemm_thin": 0 = bf16 products with at most 64 output columns over 1024 rows or
  * more go through the tiled kernels and their split-K reduce instead of the one-pass kernel for
- * thin outputs (default 1). "gemm_row_split": 0 = a product on 256x256 tiles whose last round
+ * thin outputs (default 1). "q8_widen": int8 products over a widened copy of the weight in scratch: -1 = where
+ * that is estimated to be ahead (default), 0 = never, 1 = wherever they can. "gemm_row_split": 0 = a product on 256x256 tiles whose last round
  * of tiles fills under 2/5 of the compute units is not cut into two launches by rows (default 1:
  * the rows of the whole rounds keep the tiling, the rest choose their own). "kv_attention": 0 = choose by head_dim (default), 1 = always the
  * LDS-tiled kernel. "ce_fused": 0 = the fused linear-cross-entropy always takes its separate

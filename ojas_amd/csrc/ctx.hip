@@ -169,6 +169,26 @@ void omx_release_pool(omx_ctx* ctx) {
   ctx->pooled_bytes = 0;
 }
 
+namespace {
+bool capturing(const omx_ctx* ctx) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
+// Gives workspace kExtraSlot back, unless the op that runs uses it or a graph holds its address. Whether it did.
+bool drop_extra(omx_ctx* ctx) {
+  void*& held = ctx->workspace[kExtraSlot];
+  if (!held || ctx->extra_in_use || ctx->workspace_captured[kExtraSlot] || capturing(ctx)) return false;
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  ctx->budget_live -= ctx->allocations[held];
+  ctx->allocations.erase(held);
+  (void)hipFree(held);
+  held = nullptr;
+  ctx->workspace_bytes[kExtraSlot] = 0;
+  return true;
+}
+}  // namespace
+
 extern "C" {
 
 int32_t omx_alloc(omx_ctx* ctx, uint64_t bytes, void** out) {
@@ -177,6 +197,7 @@ int32_t omx_alloc(omx_ctx* ctx, uint64_t bytes, void** out) {
   *out = nullptr;
   if (bytes == 0) return omx_fail(ctx, OMX_SHAPE, "omx_alloc: zero bytes");
   // Charge before allocating; refuse, never clamp (budget.rs:257-316).
+  if (ctx->budget_limit && bytes <= ctx->budget_limit && ctx->budget_live > ctx->budget_limit - bytes) drop_extra(ctx);
   if (ctx->budget_limit && (bytes > ctx->budget_limit || ctx->budget_live > ctx->budget_limit - bytes))
     return omx_fail(ctx, OMX_CAPACITY_EXCEEDED, "requested %llu cap %llu live %llu", (unsigned long long)bytes,
                     (unsigned long long)ctx->budget_limit, (unsigned long long)ctx->budget_live);
@@ -194,6 +215,10 @@ int32_t omx_alloc(omx_ctx* ctx, uint64_t bytes, void** out) {
       // Out of device memory with blocks parked in the pool: give them back and try once more.
       (void)hipGetLastError();
       omx_release_pool(ctx);
+      err = hipMalloc(&p, bytes);
+    }
+    if (err != hipSuccess && drop_extra(ctx)) {
+      (void)hipGetLastError();
       err = hipMalloc(&p, bytes);
     }
     if (err != hipSuccess) return omx_hip_fail(ctx, err, "hipMalloc");
@@ -298,11 +323,6 @@ int32_t omx_unsupported(omx_ctx* ctx, const char* op) {
 
 namespace {
 uint64_t workspace_size(uint64_t bytes) { return (bytes + (1ull << 20) - 1) & ~((1ull << 20) - 1); }
-
-bool capturing(const omx_ctx* ctx) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
-}
 }  // namespace
 
 bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot) {

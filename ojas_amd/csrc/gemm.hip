@@ -508,7 +508,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a_rs, uint64_t a_cs, const void* b,
                       uint64_t b_rs, uint64_t b_cs, int32_t operand_dtype, void* c, int32_t c_dtype, uint64_t ldc,
                       uint64_t m, uint64_t k, uint64_t n, int32_t accumulate, const OmxGemmEpilogue* epi,
-                      const OmxGemmBatch* batch, uint64_t a_k) {
+                      const OmxGemmBatch* batch, uint64_t a_k, const OmxLowRank* low_rank) {
   const char* op = omx_fault_name(fault_op);
   const uint64_t batches = batch ? batch->count : 1;
   if (batches == 0 || batches > 65535) return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: 1..65535 products per launch", op);
@@ -579,10 +579,10 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   // everything else (odd shapes, small outputs that need split-K) takes the 128 x 128 kernel.
   // A thin output over many rows (an adapter's rank, a gate's heads) is bound by reading A once: its
   // own kernel, which neither tiles the output nor splits K across launches.
-  const bool thin = operand_dtype == OMX_BF16 && ctx->gemm_thin && !(epi && epi->mode != OMX_EPI_NONE) &&
+  const bool thin = operand_dtype == OMX_BF16 && !low_rank && ctx->gemm_thin && !(epi && epi->mode != OMX_EPI_NONE) &&
                     omx_gemm_thin_eligible(g, a_km, b_km);
   // Few rows (a decoder's linear layers): K shared between a workgroup's waves, no tile of 128 rows.
-  const double skinny_us = operand_dtype == OMX_BF16 && !thin && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
+  const double skinny_us = operand_dtype == OMX_BF16 && !thin && !low_rank && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
                                ? omx_gemm_skinny_us(ctx, g, a_km, b_km, epi && epi->mode != OMX_EPI_NONE) : -1.0;
   bool skinny = skinny_us >= 0.0;
   int frag32 = -1, dma32 = -1;
@@ -729,12 +729,17 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       ctx->gemm_in_row_split = true;
       ctx->gemm_forced_tiling = dma_variant;
       int32_t rc = omx_gemm_impl(ctx, fault_op, a, a_rs, a_cs, b, b_rs, b_cs, operand_dtype, c, c_dtype, ldc, m0, k, n,
-                                 accumulate, epi, nullptr, a_k);
+                                 accumulate, epi, nullptr, a_k, low_rank);
       ctx->gemm_forced_tiling = -1;
+      OmxLowRank rest_rank{};
+      if (low_rank) {
+        rest_rank = *low_rank;
+        rest_rank.h = static_cast<const unsigned short*>(rest_rank.h) + m0 * rest_rank.h_pitch;
+      }
       if (rc == OMX_OK)
         rc = omx_gemm_impl(ctx, fault_op, static_cast<const char*>(a) + m0 * a_rs * esz, a_rs, a_cs, b, b_rs, b_cs,
                            operand_dtype, static_cast<char*>(c) + m0 * ldc * csz, c_dtype, ldc, m - m0, k, n,
-                           accumulate, epi, nullptr, a_k);
+                           accumulate, epi, nullptr, a_k, low_rank ? &rest_rank : nullptr);
       ctx->gemm_in_row_split = false;
       return rc;
     }
@@ -809,6 +814,16 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       if (wrc != OMX_OK) return wrc;
       g.partial = static_cast<float*>(ws);
     }
+  }
+  g.lr_rank = g.lr_block_cols = 0;
+  if (low_rank) {
+    if (dma_variant < 0) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: no kernel for a low-rank term at this shape", op);
+    g.lr_h = static_cast<const unsigned short*>(low_rank->h);
+    g.lr_w = static_cast<const unsigned short*>(low_rank->w);
+    g.lr_pitch = static_cast<long>(low_rank->h_pitch);
+    g.lr_w_pitch = static_cast<long>(low_rank->w_pitch);
+    g.lr_rank = static_cast<int>(low_rank->rank);
+    g.lr_block_cols = static_cast<int>(low_rank->block_cols);
   }
   g.epi = epi ? epi->mode : OMX_EPI_NONE;
   g.epi_tanh = epi ? epi->tanh_form : 0;
@@ -885,6 +900,27 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   return rc;
 }
 
+// What the bf16 product of a k-contiguous A takes on the direct-to-LDS tiling with the least estimate: dma_us, and for the
+// one-wave tiles rounds of tiles x (4 or 3 units per K step of 64 and 18 around them; a unit is 0.373 us: 8192 x 2048 over 8192
+// 198 us, 203 measured, 8192^3 791 and 790).
+double omx_gemm_bf16_us(const omx_ctx* ctx, uint64_t m, uint64_t k, uint64_t n) {
+  const long cus = ctx->cu_count > 0 ? ctx->cu_count : 256, rows = static_cast<long>(m), cols = static_cast<long>(n);
+  const int ksteps = static_cast<int>((k + 63) / 64);
+  double best = 1e30;
+  for (int v : {3, 6, 7, 8}) best = std::min(best, dma_us(v, rows, cols, 1, ksteps, 1, false, false, false, cus));
+  if (k % 128 == 0)
+    for (long w : {4l, 3l}) {
+      const long tiles = (rows + 255) / 256 * ((cols + 64 * w - 1) / (64 * w));
+      best = std::min(best, 0.373 * static_cast<double>((tiles + cus - 1) / cus) * (w * ksteps + 18.0));
+    }
+  return best;
+}
+
+bool omx_gemm_takes_low_rank(const omx_ctx* ctx, const void* a, uint64_t lda, const void* b, uint64_t ldb, uint64_t k) {
+  return ctx->gemm_dma_mode == 1 && k % 64 == 0 && aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 && lda < 1ull << 22 &&
+         ldb < 1ull << 22;
+}
+
 int32_t omx_timing_begin(omx_ctx* ctx, double flops, omx_ctx::TimedLaunch* timed) {
   *timed = omx_ctx::TimedLaunch{};
   if (!ctx->profile_gemm) return OMX_OK;
@@ -949,6 +985,11 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value) {
   if (name && strcmp(name, "gemm_f32") == 0) {
     if (value < -1 || value > FRAG32_TILES + DMA32_TILES) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: gemm_f32 takes -1..9");
     ctx->gemm_f32_tile = static_cast<int>(value);
+    return OMX_OK;
+  }
+  if (name && strcmp(name, "q8_widen") == 0) {
+    if (value < -1 || value > 1) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: q8_widen takes -1..1");
+    ctx->q8_widen = static_cast<int>(value);
     return OMX_OK;
   }
   if (name && strcmp(name, "gemm_row_split") == 0) {

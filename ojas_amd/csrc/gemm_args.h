@@ -23,6 +23,11 @@ struct GemmArgs {
   float epi_s1, epi_s2;  // OMX_EPI_AXPBY
   OmxFaultWord* fault;
   unsigned long long tag, act_tag;  // act_tag: of the f32 store pass's activation
+  // bf16, A k-contiguous: C[m, n] += sum_p lr_h[m][off + p] lr_w[n][p] in the accumulators, p < lr_rank (a multiple of 16; 0:
+  // none), off = n / lr_block_cols * lr_rank where lr_block_cols (a multiple of 32) is not 0. Pitches in elements.
+  const unsigned short *lr_h, *lr_w;
+  long lr_pitch, lr_w_pitch;
+  int lr_rank, lr_block_cols;
   // Strided batch: block (x, y) works on product y, whose operands start batch_* BYTES after
   // product y - 1's. batches == 1 for a single product.
   int batches;

@@ -8,7 +8,8 @@
 namespace {
 
 // EPI: the store pass (OMX_EPI_*). A kernel of its own per store pass keeps each one's code (a few KiB of
-// straight-line stores) and registers out of the others. TAIL: see StepBase.
+// straight-line stores) and registers out of the others; EPI_LOW_RANK is the plain one behind a low-rank term. TAIL: see StepBase.
+constexpr int EPI_LOW_RANK = 16;
 template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI, bool TAIL = false>
 __global__ __launch_bounds__(WGM* WGN * 64, dma_waves_per_simd(WGM* WGN, NST*(WGM* TM + WGN * TN) * 32 * DBK * 2)) void
 gemm_dma_kernel(GemmArgs g) {
@@ -167,6 +168,13 @@ gemm_dma_kernel(GemmArgs g) {
       st = nx;
     }
   }
+  if constexpr (EPI == EPI_LOW_RANK) {
+    if (split == 0)
+      gemm_low_rank<TM, TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32, lane, [&](auto t, auto u, const u32x4& a, const u32x4& b) {
+        floatx16& c = acc[decltype(t)::value][decltype(u)::value];
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+      });
+  }
   __syncthreads();  // the staging below reuses the stages
 
   // Epilogue: each wave stages 32 rows of its tile at a time through its own
@@ -193,7 +201,7 @@ gemm_dma_kernel(GemmArgs g) {
     bool stored = false;
     if constexpr (kFastStores) {
       const bool interior = grow0 + 32 <= g.M && gcol0 + TN * 32 <= g.N;
-      if constexpr (EPI == OMX_EPI_NONE) {
+      if constexpr (EPI == OMX_EPI_NONE || EPI == EPI_LOW_RANK) {
         if (interior && (g.splits > 1 ? (g.N & 3) == 0 : g.c_vec != 0)) {
           if (g.splits > 1) bad |= gemm_store_block<0, PPR>(g, split, cs, CPW, grow0, gcol0, lane);
           else if (g.c_bf16) bad |= gemm_store_block<1, PPR>(g, split, cs, CPW, grow0, gcol0, lane);
@@ -207,7 +215,7 @@ gemm_dma_kernel(GemmArgs g) {
           bad |= gemm_epilogue_block<OMX_EPI_AXPBY, false, PPR>(g, cs, CPW, grow0, gcol0, lane);
           stored = true;
         }
-      } else if constexpr (EPI != OMX_EPI_NONE) {
+      } else if constexpr (EPI != OMX_EPI_NONE && EPI != EPI_LOW_RANK) {
         if (interior && g.c_vec != 0) {
           bad |= g.epi_tanh ? gemm_epilogue_block<EPI, true, PPR>(g, cs, CPW, grow0, gcol0, lane)
                             : gemm_epilogue_block<EPI, false, PPR>(g, cs, CPW, grow0, gcol0, lane);
@@ -245,6 +253,9 @@ int32_t launch_dma(omx_ctx* ctx, const GemmArgs& g) {
   // (gemm_dma.hip takes a ragged reduction only with the plain store pass)
   if constexpr (B_KM) {
     if (g.k_rows != g.K) kernel = &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_NONE, true>;
+  }
+  if constexpr (!A_KM) {
+    if (g.lr_rank > 0) kernel = &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, EPI_LOW_RANK>;  // (whole steps)
   }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    smem));

@@ -8,7 +8,7 @@
 //
 // Data movement, per workgroup (512 threads, tile 256 x 128, 32-column K steps):
 //   * the activation operand goes global -> LDS directly, three stages, as in gemm_dma.hip;
-//   * the codes never exist as bf16 in HBM: waves 0..3 each fetch 1 KiB of codes per step
+//   * the codes are widened on their way (widened_product does it in memory, where that is ahead): waves 0..3 each fetch 1 KiB of codes per step
 //     (global -> LDS directly, 16 codes per lane) plus the lane's group scale, three steps ahead;
 //     the wave that fetched them reads its own 16 bytes back, widens them
 //     (fma(byte ^ 0x80, scale, -128 scale) is code * scale rounded once, then round-to-nearest-even
@@ -19,6 +19,8 @@
 //     scales = 79 KiB: two workgroups share a compute unit.
 // HBM traffic per product: the activation once per column band, the codes once per row band at
 // ONE byte per weight, the scales at one eighth of that.
+#include <algorithm>
+
 #include "gemm_tiles.h"
 
 typedef __bf16 bf16x2q __attribute__((ext_vector_type(2)));
@@ -392,6 +394,38 @@ __global__ void q8_pack_kernel(const signed char* __restrict__ src, const float*
   }
 }
 
+// The weight as bf16, row-major: what gemm_q8_kernel widens a tile at a time. A thread takes 16 codes, eight of them the 128
+// columns of a block's row.
+__global__ void q8_widen_kernel(const signed char* __restrict__ codes, const float* __restrict__ scales,
+                                unsigned short* __restrict__ out, long nout, long kin, int packed) {
+  const long pieces = nout * (kin / 16);
+  const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= pieces) return;
+  long row, p;
+  if (packed) {
+    const long block = i >> 6, across = kin >> 7;
+    row = block / across * 8 + ((i >> 3) & 7);
+    p = block % across * 8 + (i & 7);
+  } else {
+    row = i / (kin / 16);
+    p = i % (kin / 16);
+  }
+  const long group = p >> 1;
+  const uint4 v = *reinterpret_cast<const uint4*>(codes + (packed ? q8_packed_code_offset(row, group, kin) + (p & 1) * 16 : row * kin + p * 16));
+  const float s = scales[packed ? q8_packed_scale_index(row, group, kin) : row * (kin / 32) + group];
+  const unsigned w[4] = {v.x, v.y, v.z, v.w};
+  unsigned r[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      r[2 * j + h] = q8_pack2(static_cast<float>(static_cast<signed char>(w[j] >> (16 * h))) * s,
+                              static_cast<float>(static_cast<signed char>(w[j] >> (16 * h + 8))) * s);
+  uint4* to = reinterpret_cast<uint4*>(out + row * kin + p * 16);
+  to[0] = make_uint4(r[0], r[1], r[2], r[3]);
+  to[1] = make_uint4(r[4], r[5], r[6], r[7]);
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 template <bool B_KM>
@@ -461,6 +495,43 @@ int32_t set_low_rank(omx_ctx* ctx, const char* op, Q8Args* g, const omx_low_rank
   return OMX_OK;
 }
 
+// Whether the product takes less over a copy of the weight widened into scratch (as many bytes again as its codes, twice) than over
+// the codes. gemm_q8_kernel's widening rides on four of eight waves and holds it at 950 TFLOP/s, one tiling whatever the shape;
+// the bf16 kernels do 1070 to 1360 on the same products and have small tiles for small ones, and give the same bits. Estimates in
+// us: a 32-column step of gemm_q8_kernel 0.46 alone on a compute unit, 1.06 with two there; the copy 3.5 and 3.1 bytes a weight
+// at 4.5 TB/s. us over codes and over the copy, forward / input gradient: 8192 rows over 2048 x 16384: 590, 525 / 552, 421; over
+// 2048 x 2048: 77, 70 / 76, 65; 1024 rows there: 34, 26 / 37, 27; 64 rows over 2048 x 6144: 35, 25 / 100, 25. The other way round,
+// and left: 8192 rows over 512 -> 4096: 49, 58; 512 over 2048 -> 16384: 48, 64.
+bool widen_pays(const omx_ctx* ctx, uint64_t m, uint64_t k, uint64_t n) {
+  if (ctx->q8_widen >= 0) return ctx->q8_widen != 0;
+  const double cus = ctx->cu_count > 0 ? ctx->cu_count : 256, tiles = static_cast<double>((m + QBM - 1) / QBM * ((n + QBN - 1) / QBN));
+  const double over_codes = 4.0 + static_cast<double>(k / QBK) * (tiles <= cus ? 0.46 : 1.06 * std::max(1.0, tiles / (2.0 * cus)));
+  const double over_copy = 3.5 + static_cast<double>(k) * static_cast<double>(n) * 6.9e-7 + omx_gemm_bf16_us(ctx, m, k, n);
+  return over_copy < 0.93 * over_codes;
+}
+int32_t widened_product(omx_ctx* ctx, uint32_t fault_op, const Q8Args& g, uint64_t rows, uint64_t kin, uint64_t nout,
+                        bool backward, bool* taken) {
+  *taken = false;
+  const uint64_t k = backward ? nout : kin, n = backward ? kin : nout;
+  constexpr uint64_t kMost = 1ull << 30;  // bytes of scratch
+  if (g.add || nout * kin * 2 > kMost || !widen_pays(ctx, rows, k, n) || !omx_gemm_takes_low_rank(ctx, g.a, k, nullptr, kin, k)) return OMX_OK;
+  unsigned short* w = static_cast<unsigned short*>(omx_workspace_if_room(ctx, nout * kin * 2, kExtraSlot));
+  if (!w) return OMX_OK;
+  const long pieces = static_cast<long>(nout) * static_cast<long>(kin / 16);
+  omx_launch(ctx, q8_widen_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, g.codes, g.scales, w,
+             static_cast<long>(nout), static_cast<long>(kin), g.packed);
+  OMX_LAUNCH_CHECK(ctx, "q8_widen_kernel");
+  const OmxLowRank lr{g.lr_h, g.lr_w, static_cast<uint64_t>(g.lr_pitch), static_cast<uint64_t>(g.lr_w_pitch),
+                      static_cast<uint64_t>(g.lr_rank), static_cast<uint64_t>(g.lr_block_cols)};
+  ctx->extra_in_use = true;
+  const int32_t rc = omx_gemm_impl(ctx, fault_op, g.a, k, 1, w, backward ? kin : 1, backward ? 1 : kin, OMX_BF16, g.c,
+                                   g.c_f32 ? OMX_F32 : OMX_BF16, n, rows, k, n, 0, nullptr, nullptr, 0, g.lr_rank > 0 ? &lr : nullptr);
+  ctx->extra_in_use = false;
+  // Partial sums that there is no room for: the codes' kernel has none.
+  *taken = rc != OMX_CAPACITY_EXCEEDED;
+  return *taken ? rc : OMX_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -494,6 +565,9 @@ int32_t omx_linear_i8_group_forward(omx_ctx* ctx, const void* x, int32_t x_dtype
   g.fault = ctx->fault;
   rc = set_low_rank(ctx, op, &g, low_rank, nout);
   if (rc != OMX_OK) return rc;
+  bool taken = false;
+  rc = widened_product(ctx, F_LINEAR_FORWARD, g, rows, kin, nout, false, &taken);
+  if (rc != OMX_OK || taken) return rc;
   g.tag = omx_tag(ctx, F_LINEAR_FORWARD);
   return launch_q8<false>(ctx, g, 2.0 * rows * kin * nout);
 }
@@ -526,6 +600,9 @@ int32_t omx_linear_i8_group_backward_input(omx_ctx* ctx, const void* codes_i8, c
   g.fault = ctx->fault;
   rc = set_low_rank(ctx, op, &g, low_rank, kin);
   if (rc != OMX_OK) return rc;
+  bool taken = false;
+  rc = widened_product(ctx, F_LINEAR_BACKWARD, g, rows, kin, nout, true, &taken);
+  if (rc != OMX_OK || taken) return rc;
   g.tag = omx_tag(ctx, F_LINEAR_BACKWARD);
   return launch_q8<true>(ctx, g, 2.0 * rows * kin * nout);
 }

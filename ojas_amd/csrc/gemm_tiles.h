@@ -205,6 +205,25 @@ __device__ __forceinline__ void wait_loads(int groups) {
   }
 }
 
+// The low-rank term of a wave's TM x TN blocks of 32 x 32 from (row0, col0) on, its operands straight from memory into fragments
+// (a few KiB a row block): product(t, u, a, b) multiplies 16 columns of it into block (t, u).
+template <int TM, int TN, typename P>
+__device__ __forceinline__ void gemm_low_rank(const GemmArgs& g, int row0, int col0, int lane, P product) {
+  const int l32 = lane & 31, lg = lane >> 5;
+#pragma unroll 1
+  for (int p = 0; p < g.lr_rank; p += 16)
+    static_for<0, TN>([&](auto u_index) {
+      constexpr int u = decltype(u_index)::value;
+      const int col = min(col0 + u * 32, g.N - 1);
+      const unsigned short* h = g.lr_h + p + 8 * lg + (g.lr_block_cols > 0 ? col / g.lr_block_cols * g.lr_rank : 0);
+      const u32x4 b = *reinterpret_cast<const u32x4*>(g.lr_w + min(col0 + u * 32 + l32, g.N - 1) * g.lr_w_pitch + p + 8 * lg);
+      static_for<0, TM>([&](auto t_index) {
+        constexpr int t = decltype(t_index)::value;
+        product(t_index, u_index, *reinterpret_cast<const u32x4*>(h + min(row0 + t * 32 + l32, g.M - 1) * g.lr_pitch), b);
+      });
+    });
+}
+
 // Waves per SIMD the kernel is compiled for: as many workgroups per compute unit as its LDS (160
 // KiB) allows, up to four waves per SIMD.
 constexpr int dma_waves_per_simd(int waves, int lds_bytes) {

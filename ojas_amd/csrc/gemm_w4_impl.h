@@ -121,7 +121,8 @@ struct W4Frags {
   }
 };
 
-template <bool A_KM, bool B_KM, int TN, bool TAIL>
+// LR: with a low-rank term.
+template <bool A_KM, bool B_KM, int TN, bool TAIL, bool LR = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   static_assert(!A_KM || B_KM, "a k-major A goes with a k-major B");
   static_assert(TN == 4 || TN == 3, "256 x 256 or 256 x 192 tiles");
@@ -416,6 +417,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
       step(S1, j + 2 < steps, j + 3 < steps);
     }
   }
+  if constexpr (LR) {
+    if (split == 0)
+      gemm_low_rank<TM, TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32, lane, [&](auto t, auto u, const u32x4& a, const u32x4& b) {
+        product_of(acc[decltype(t)::value][decltype(u)::value], a, b);
+      });
+  }
   // Every wave has read its last fragments before the stages are reused for the store pass.
   __builtin_amdgcn_s_waitcnt(vmcnt_only(0) & 0xC07F);
   __builtin_amdgcn_s_barrier();
@@ -505,6 +512,9 @@ int32_t launch_w4(omx_ctx* ctx, const GemmArgs& g) {
   auto kernel = &gemm_w4_kernel<A_KM, B_KM, TN, false>;
   if constexpr (B_KM) {
     if (g.k_rows != g.K) kernel = &gemm_w4_kernel<A_KM, B_KM, TN, true>;
+  }
+  if constexpr (!A_KM) {
+    if (g.lr_rank > 0) kernel = &gemm_w4_kernel<A_KM, B_KM, TN, false, true>;  // (whole steps)
   }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    W4_SMEM));

@@ -85,9 +85,10 @@ struct omx_ctx {
   // Slot 0: per-op scratch. Slot 1: split-K partials of the GEMM (which an op
   // may call while it holds slot 0) and operands converted for an op that holds slot 0.
   // Slot 2: tensors an op keeps across calls into other ops (a recomputed attention output).
-  void* workspace[3] = {nullptr, nullptr, nullptr};
-  uint64_t workspace_bytes[3] = {0, 0, 0};
-  bool workspace_captured[3] = {false, false, false};  // handed out while the stream was captured
+  void* workspace[4] = {nullptr, nullptr, nullptr, nullptr};
+  uint64_t workspace_bytes[4] = {0, 0, 0, 0};
+  bool extra_in_use = false;  // workspace kExtraSlot, by the op that runs
+  bool workspace_captured[4] = {false, false, false, false};  // handed out while the stream was captured
   int cu_count = 0;
   // This device's copy of the static scratch of omx_cross_entropy_mean_forward_static, looked up
   // when the context is opened (the lookup is not stream work and may load the code object).
@@ -95,6 +96,7 @@ struct omx_ctx {
   // Optional per-launch timing of the GEMM kernel (benchmark only).
   // 0: 128x128 register-staged kernel only; 1: choose by shape; others force a direct-to-LDS tiling (omx_set_option).
   int gemm_dma_mode = 1;
+  int q8_widen = -1;         // int8 products over a widened copy of the weight: -1 by rule, 0 never, 1 wherever they can
   int gemm_f32_tile = -1;    // f32 products: -1: choose by estimate; 0..4, 5..8: a tile of gemm_frag32.hip, gemm_dma32.hip; 9: the register-staged kernel
   int gemm_row_split = 1;    // 0: a product whose last round of 256 x 256 tiles is mostly empty is not cut by rows
   bool gemm_in_row_split = false;  // set while omx_gemm_impl runs the two halves of a cut product
@@ -183,6 +185,8 @@ struct OmxKernelTimer {
 };
 
 int32_t omx_hip_fail(omx_ctx* ctx, hipError_t err, const char* what);
+// Workspace kExtraSlot is for what an op can do without: any allocation that would be refused takes it back first.
+constexpr int kExtraSlot = 3;
 // Grows workspace `slot` to at least `bytes` (budget-charged).
 int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot = 0);
 // Whether the budget has room for workspace `slot` at that size (for an op that can do with less).
@@ -205,6 +209,11 @@ inline unsigned long long omx_tag(omx_ctx* ctx, uint32_t op) {
 //     s2 A.B, each term rounded as a pass of its own would.
 // aux tensors have C's layout (pitch, and batch stride in a strided batch).
 enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3 };
+// A term of small rank beside a bf16 product, added in its accumulators (GemmArgs: lr_*).
+struct OmxLowRank {
+  const void *h, *w;
+  uint64_t h_pitch, w_pitch, rank, block_cols;
+};
 struct OmxGemmEpilogue {
   int mode;
   int tanh_form;
@@ -220,7 +229,10 @@ struct OmxGemmBatch {
 int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a_rs, uint64_t a_cs, const void* b,
                       uint64_t b_rs, uint64_t b_cs, int32_t operand_dtype, void* c, int32_t c_dtype, uint64_t ldc,
                       uint64_t m, uint64_t k, uint64_t n, int32_t accumulate, const OmxGemmEpilogue* epi = nullptr,
-                      const OmxGemmBatch* batch = nullptr, uint64_t a_k = 0);
+                      const OmxGemmBatch* batch = nullptr, uint64_t a_k = 0, const OmxLowRank* low_rank = nullptr);
+double omx_gemm_bf16_us(const omx_ctx* ctx, uint64_t m, uint64_t k, uint64_t n);
+// Whether omx_gemm_impl takes a bf16 product k-contiguous in A with a low-rank term (on the direct-to-LDS kernels).
+bool omx_gemm_takes_low_rank(const omx_ctx* ctx, const void* a, uint64_t lda, const void* b, uint64_t ldb, uint64_t k);
 // out[c] = sum over b < blocks of partial[b * dim + c], added in a fixed order.
 // `scratch` (OMX_COLUMN_SUM_GROUPS * dim floats, may be null) lets a tall `partial` be added in two stages.
 constexpr int OMX_COLUMN_SUM_GROUPS = 32;

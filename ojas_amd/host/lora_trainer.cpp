@@ -9,7 +9,7 @@
 // Layout choices:
 //  * q, k, v share one fused projection [3d, d] and gate, up one [2 hidden, d], so a block has four
 //    quantised products each way; the base matrices live in the blocked int8 layout
-//    (omx_pack_i8_group) and are never widened in memory.
+//    (omx_pack_i8_group) and are widened in memory one at a time at most.
 //  * The adapters live in one f32 arena, every A of every layer first ([Aq, Ak, Av, Ao] per layer,
 //    so a layer's q, k, v down-projections are one [3r, d] matrix), then every B ([Bq, Bk, Bv, Bo]
 //    per layer: the three up-projections stacked are the [3d, r] operand of the fused

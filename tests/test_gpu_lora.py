@@ -72,6 +72,41 @@ def test_linear_i8_group_backward_input(be, rows, kin, nout, with_add):
     _close(be.download_f32(gx), want)
 
 
+# Rows: under and around a tile; k_in and n_out: one step and ragged tiles; (rank, block_cols) of the low-rank term.
+@pytest.mark.parametrize("backward", [False, True])
+@pytest.mark.parametrize("rows,kin,nout,rank,block,blocked", [
+    (33, 128, 64, 16, 0, True), (257, 128, 384, 16, 128, True), (1025, 512, 768, 32, 256, True), (300, 192, 320, 16, 0, False),
+    (4100, 256, 512, 0, 0, True), (8193, 768, 2304, 16, 768, True)])
+def test_linear_i8_group_over_a_widened_copy(be, rows, kin, nout, rank, block, blocked, backward):
+    # A weight widened in scratch gives the bits of one widened on its way: the same bf16 values, the same order of sums.
+    from ojas_amd.backend import BF16, F32
+
+    print(f"q8 widened rows={rows} kin={kin} nout={nout} rank={rank} backward={backward}", flush=True)
+    rng = np.random.default_rng(rows + kin)
+    codes = be.upload(rng.integers(-127, 128, (nout, kin)).astype(np.int8))
+    scales = be.upload(rng.uniform(1e-4, 1e-3, (nout, kin // 32)).astype(np.float32))
+    if blocked:
+        codes, scales = be.pack_i8_group(codes, scales)
+    cols = kin if backward else nout
+    if backward:
+        block = 0
+    x = be.upload(rng.normal(0, 1, (rows, nout if backward else kin)).astype(np.float32), BF16)
+    low_rank = None
+    if rank:
+        h = rng.normal(0, 1, (rows, rank * (cols // block if block else 1))).astype(np.float32)
+        low_rank = (be.upload(h, BF16), be.upload(rng.normal(0, 0.1, (cols, rank)).astype(np.float32), BF16), block)
+    got = []
+    try:
+        for widen in (0, 1):
+            be.set_option("q8_widen", widen)
+            y = (be.linear_i8_group_backward_input(codes, scales, x, blocked=blocked, low_rank=low_rank) if backward else
+                 be.linear_i8_group_forward(x, codes, scales, blocked=blocked, low_rank=low_rank, out_dtype=F32))
+            got.append(be.download_f32(y))
+    finally:
+        be.set_option("q8_widen", -1)
+    assert np.array_equal(got[0], got[1])
+
+
 def test_linear_i8_group_scale_per_group_is_exact(be):
     # One code per group set, powers of two as scales, a one-hot input: the product is exact in
     # bf16, so a scale taken from the wrong group or row, or a mis-signed code, shows bit for bit.

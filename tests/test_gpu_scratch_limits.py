@@ -234,3 +234,28 @@ def test_gate_backward_with_room_for_fewer_partial_rows():
     got = with_less(lambda be, *t: be.per_head_sigmoid_gate_backward(*t), [x, w, b, attn, gy], 1)
     for a, c in zip(got, orc.gate_backward(x, w, b, attn, gy)):
         close(a, c)
+
+
+def test_a_widened_weight_makes_room_for_what_is_allocated_next():
+    # 2 MiB of bf16 weight in scratch; the budget then has room for the next tensor only without it.
+    from ojas_amd.backend import BF16, F32, MiBackend
+
+    rng = np.random.default_rng(3)
+    x, codes = rng.normal(0, 1, (512, 1024)).astype(np.float32), rng.integers(-127, 128, (1024, 1024)).astype(np.int8)
+    scales = rng.uniform(1e-4, 1e-3, (1024, 32)).astype(np.float32)
+    be = MiBackend(0, budget_bytes=16 << 20)
+    try:
+        dx, dc, ds = be.upload(x, BF16), be.upload(codes), be.upload(scales)
+        be.set_option("q8_widen", 0)
+        want = be.download_f32(be.linear_i8_group_forward(dx, dc, ds))
+        be.set_option("q8_widen", 1)
+        held = be.budget()["live"]
+        y = be.linear_i8_group_forward(dx, dc, ds)
+        assert be.budget()["live"] - held >= 2 << 20
+        rest = be.empty(((16 << 20) - be.budget()["live"] + (1 << 20)) // 4, F32)  # a MiB more than there is
+        assert np.array_equal(be.download_f32(y), want)
+        z = be.linear_i8_group_forward(dx, dc, ds)  # no room for the copy
+        assert np.array_equal(be.download_f32(z), want)
+        del rest
+    finally:
+        be.close()
