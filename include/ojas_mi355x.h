@@ -327,6 +327,14 @@ int32_t omx_rms_norm_backward_residual(omx_ctx* ctx, const void* x, int32_t x_dt
                                        const void* w_f32, const void* gy, int32_t gy_dtype,
                                        const void* residual_grad_f32, void* gx_f32, void* gx_bf16,
                                        void* gw_f32, uint64_t rows, uint64_t dim, float eps);
+/* From here on the weight gradients of rms_norm_backward and _residual and the bias gradients of
+ * per_head_sigmoid_gate_backward and _deferred may wait, until omx_form_weight_sums forms them (`form` = 0: forgets them), as few
+ * launches: each is a sum over some hundred partial rows, and a launch of its own takes 4 to 5 us whatever its size. Their
+ * outputs are written by then, with the same bits; a non-finite one is reported under the op that it belongs to. `expected`: how many,
+ * for the size of the scratch (at most 64 MiB, given back to any allocation that would be refused once nothing waits); without
+ * room they are formed at once. The reference's tape forms each where it stands (ojas-autograd/src/tape.rs:2565-2591). */
+int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected);
+int32_t omx_form_weight_sums(omx_ctx* ctx, int32_t form);
 
 /* ---- BackendModule::cross_entropy_mean_forward / _backward
  *      (backend.rs:2451-2466). loss is one f32 on the device. ---- */

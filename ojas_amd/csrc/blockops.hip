@@ -636,7 +636,8 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
     gates = fresh;
   }
   void* gz = gz_out ? gz_out : static_cast<void*>(base + gates_bytes);
-  float* partial = reinterpret_cast<float*>(base + gates_bytes + gz_bytes);
+  float* waiting = omx_partial_rows(ctx, blocks, heads);
+  float* partial = waiting ? waiting : reinterpret_cast<float*>(base + gates_bytes + gz_bytes);
   float* stage = reinterpret_cast<float*>(base + gates_bytes + gz_bytes + partial_bytes);
 
   const bool vec = head_dim % 4 == 0 && packs_of_four(4, omx_dtype_size(attn_dtype), {attn, gy}) &&
@@ -673,7 +674,7 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
 #undef GATE_BWD_V
 #undef GATE_BWD
   OMX_LAUNCH_CHECK(ctx, "gate_bwd_kernel");
-  rc = omx_column_sum(ctx, partial, static_cast<float*>(g_bias), blocks, heads, tag, stage);
+  rc = omx_column_sum(ctx, partial, static_cast<float*>(g_bias), blocks, heads, tag, stage, nullptr, waiting != nullptr);
   if (rc != OMX_OK) return rc;
   // grad_input[r, i] = sum_h gz[r, h] weight[h, i]
   if (g_input) {

@@ -175,17 +175,23 @@ bool capturing(const omx_ctx* ctx) {
   return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 
-// Gives workspace kExtraSlot back, unless the op that runs uses it or a graph holds its address. Whether it did.
+// Gives workspaces kExtraSlot and kSumsSlot back, unless the op that runs or sums that wait use them or a graph holds their
+// address. Whether there was one.
 bool drop_extra(omx_ctx* ctx) {
-  void*& held = ctx->workspace[kExtraSlot];
-  if (!held || ctx->extra_in_use || ctx->workspace_captured[kExtraSlot] || capturing(ctx)) return false;
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
-  ctx->budget_live -= ctx->allocations[held];
-  ctx->allocations.erase(held);
-  (void)hipFree(held);
-  held = nullptr;
-  ctx->workspace_bytes[kExtraSlot] = 0;
-  return true;
+  bool dropped = false;
+  for (int slot : {kExtraSlot, kSumsSlot}) {
+    void*& held = ctx->workspace[slot];
+    const bool in_use = slot == kExtraSlot ? ctx->extra_in_use : !ctx->sums.empty();
+    if (!held || in_use || ctx->workspace_captured[slot] || capturing(ctx)) continue;
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return dropped;
+    ctx->budget_live -= ctx->allocations[held];
+    ctx->allocations.erase(held);
+    (void)hipFree(held);
+    held = nullptr;
+    ctx->workspace_bytes[slot] = 0;
+    dropped = true;
+  }
+  return dropped;
 }
 }  // namespace
 

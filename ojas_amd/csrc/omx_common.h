@@ -67,6 +67,14 @@ struct OmxFaultWord {
   unsigned long long first;  // (sequence << 8) | op, ~0 when clear
 };
 
+// out[c] = sum over b < blocks of partial[b * dim + c].
+struct OmxColumnSum {
+  const float* partial;
+  float* out;
+  unsigned long long tag;
+  int blocks, dim;
+};
+
 struct omx_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -85,10 +93,15 @@ struct omx_ctx {
   // Slot 0: per-op scratch. Slot 1: split-K partials of the GEMM (which an op
   // may call while it holds slot 0) and operands converted for an op that holds slot 0.
   // Slot 2: tensors an op keeps across calls into other ops (a recomputed attention output).
-  void* workspace[4] = {nullptr, nullptr, nullptr, nullptr};
-  uint64_t workspace_bytes[4] = {0, 0, 0, 0};
+  void* workspace[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  uint64_t workspace_bytes[5] = {0, 0, 0, 0, 0};
   bool extra_in_use = false;  // workspace kExtraSlot, by the op that runs
-  bool workspace_captured[4] = {false, false, false, false};  // handed out while the stream was captured
+  // Column sums that wait (omx_defer_weight_sums), their partial rows in workspace kSumsSlot up to sums_used.
+  bool sums_wait = false;
+  uint32_t sums_expected = 0;
+  uint64_t sums_used = 0;
+  std::vector<OmxColumnSum> sums;
+  bool workspace_captured[5] = {false, false, false, false, false};  // handed out while the stream was captured
   int cu_count = 0;
   // This device's copy of the static scratch of omx_cross_entropy_mean_forward_static, looked up
   // when the context is opened (the lookup is not stream work and may load the code object).
@@ -185,8 +198,8 @@ struct OmxKernelTimer {
 };
 
 int32_t omx_hip_fail(omx_ctx* ctx, hipError_t err, const char* what);
-// Workspace kExtraSlot is for what an op can do without: any allocation that would be refused takes it back first.
-constexpr int kExtraSlot = 3;
+// Workspaces kExtraSlot and kSumsSlot are for what an op can do without: any allocation that would be refused takes them back first.
+constexpr int kExtraSlot = 3, kSumsSlot = 4;
 // Grows workspace `slot` to at least `bytes` (budget-charged).
 int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot = 0);
 // Whether the budget has room for workspace `slot` at that size (for an op that can do with less).
@@ -238,8 +251,11 @@ bool omx_gemm_takes_low_rank(const omx_ctx* ctx, const void* a, uint64_t lda, co
 constexpr int OMX_COLUMN_SUM_GROUPS = 32;
 // Up to this many rows a tall sum is one launch of 1024-thread workgroups.
 constexpr int OMX_COLUMN_SUM_WIDE_ROWS = 1024;
-int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t blocks, uint64_t dim,
-                       unsigned long long tag, float* scratch = nullptr, hipEvent_t stop = nullptr);
+// Sums wait in a list (`wait`) where omx_partial_rows has said so.
+int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t blocks, uint64_t dim, unsigned long long tag,
+                       float* scratch = nullptr, hipEvent_t stop = nullptr, bool wait = false);
+// Where sums wait and there is room, memory for their partial rows; else null.
+float* omx_partial_rows(omx_ctx* ctx, uint64_t blocks, uint64_t dim);
 // RMSNorm with 16-byte accesses for row widths 256..2048 (rmsvec.hip). `add` (forward) and
 // `add_in` / `gx16` (backward) are optional fused operands.
 bool omx_rms_vec_eligible(uint64_t dim, std::initializer_list<const void*> ptrs);

@@ -370,8 +370,9 @@ int32_t omx_rms_backward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const
   while (rows_per_block < (dim > 1024 ? 16 : 32) && rows / rows_per_block > 512) rows_per_block *= 2;
   const uint64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
   // A null gw: the weight is frozen, its gradient is not formed (no partial sums, no second launch).
-  float *partial = nullptr, *scratch = nullptr;
-  if (gw) {
+  float *partial = gw ? omx_partial_rows(ctx, blocks, dim) : nullptr, *scratch = nullptr;
+  const bool wait = partial != nullptr;
+  if (gw && !wait) {
     void* ws = nullptr;
     int32_t rc = omx_workspace(ctx, (blocks + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float), &ws);
     if (rc != OMX_OK) return rc;
@@ -393,12 +394,12 @@ int32_t omx_rms_backward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const
   do {                                                                                                               \
     if (full)                                                                                                        \
       omx_launch_timed(ctx, rms_bwd_vec_kernel<TX, TG, TO, N, (N > 4), true>, grid, block, smem, timer.start(),      \
-                       gw ? nullptr : timer.stop(), static_cast<const TX*>(x), w, static_cast<const TG*>(gy), add_in,                    \
+                       gw && !wait ? nullptr : timer.stop(), static_cast<const TX*>(x), w, static_cast<const TG*>(gy), add_in,                    \
                        static_cast<TO*>(gx), static_cast<h16*>(gx16), partial, static_cast<size_t>(rows),            \
                        static_cast<int>(dim), eps, rows_per_block, ctx->fault, tag);                                 \
     else                                                                                                             \
       omx_launch_timed(ctx, rms_bwd_vec_kernel<TX, TG, TO, N, (N > 4), false>, grid, block, smem, timer.start(),     \
-                       gw ? nullptr : timer.stop(), static_cast<const TX*>(x), w, static_cast<const TG*>(gy), add_in,                    \
+                       gw && !wait ? nullptr : timer.stop(), static_cast<const TX*>(x), w, static_cast<const TG*>(gy), add_in,                    \
                        static_cast<TO*>(gx), static_cast<h16*>(gx16), partial, static_cast<size_t>(rows),            \
                        static_cast<int>(dim), eps, rows_per_block, ctx->fault, tag);                                 \
   } while (0)
@@ -428,7 +429,7 @@ int32_t omx_rms_backward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const
 #undef RV_BWD
   OMX_LAUNCH_CHECK(ctx, "rms_bwd_vec_kernel");
   if (!gw) return OMX_OK;
-  return omx_column_sum(ctx, partial, gw, blocks, dim, tag, scratch, timer.stop());
+  return omx_column_sum(ctx, partial, gw, blocks, dim, tag, scratch, timer.stop(), wait);
 }
 
 extern "C" {

@@ -155,9 +155,8 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const float* __restrict
 
 // The same for tens to a few hundred rows in one launch: 16 row groups of 64 columns (1024 threads), four
 // loads in flight per thread, the groups added in a fixed order.
-__global__ __launch_bounds__(1024) void column_sum_wide_kernel(const float* __restrict__ partial,
-                                                               float* __restrict__ out, int blocks, int dim,
-                                                               OmxFaultWord* fault, unsigned long long tag) {
+__device__ __forceinline__ void column_sum_wide(const float* __restrict__ partial, float* __restrict__ out, int blocks, int dim,
+                                                OmxFaultWord* fault, unsigned long long tag) {
   __shared__ float red[16][64];
   const int lane = threadIdx.x & 63, group = threadIdx.x >> 6;
   const int c = blockIdx.x * 64 + lane;
@@ -182,6 +181,24 @@ __global__ __launch_bounds__(1024) void column_sum_wide_kernel(const float* __re
     out[c] = total;
     if (!dev_finite(total)) dev_raise_fault(fault, tag);
   }
+}
+__global__ __launch_bounds__(1024) void column_sum_wide_kernel(const float* __restrict__ partial,
+                                                               float* __restrict__ out, int blocks, int dim,
+                                                               OmxFaultWord* fault, unsigned long long tag) {
+  column_sum_wide(partial, out, blocks, dim, fault, tag);
+}
+
+// Many of them in one launch. One is 4 to 18 workgroups that wait for memory, 4 to 5 us whatever its size; the norms' of a
+// backward together take about as long as one (a step with nine norms over 2048 x 256: 1233 -> 1212 us; with thirteen over 3500 x 512:
+// 2373 -> 2346).
+constexpr int SUM_LIST = 64;
+struct ColumnSumList {
+  OmxColumnSum of[SUM_LIST];  // (2 KiB of kernel arguments)
+};
+__global__ __launch_bounds__(1024) void column_sum_list_kernel(ColumnSumList list, OmxFaultWord* fault) {
+  const OmxColumnSum& s = list.of[blockIdx.y];
+  if (static_cast<int>(blockIdx.x) * 64 >= s.dim) return;
+  column_sum_wide(s.partial, s.out, s.blocks, s.dim, fault, s.tag);
 }
 
 // Stage 1 of a tall column sum: block (x, g) adds rows [g * per_group, (g + 1) * per_group) of its
@@ -769,7 +786,11 @@ bool finite_host(float v) { return v == v && v != INFINITY && v != -INFINITY; }
 }  // namespace
 
 int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t blocks, uint64_t dim,
-                       unsigned long long tag, float* scratch, hipEvent_t stop) {
+                       unsigned long long tag, float* scratch, hipEvent_t stop, bool wait) {
+  if (wait) {
+    ctx->sums.push_back({partial, out, tag, static_cast<int>(blocks), static_cast<int>(dim)});
+    return OMX_OK;
+  }
   const unsigned col_blocks = static_cast<unsigned>((dim + 63) / 64);
   // Sixteen rows at once from 17 rows on (four at a time, each waiting for the one before, 128 rows of 256 columns took
   // 9.2 us, now 2.9).
@@ -794,7 +815,64 @@ int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t 
   return OMX_OK;
 }
 
+namespace {
+// Forms every sum that waits, in the kernel's order of rows; its partial rows' memory is free again behind it.
+int32_t form_sums(omx_ctx* ctx) {
+  for (size_t first = 0; first < ctx->sums.size(); first += SUM_LIST) {
+    ColumnSumList list{};
+    const size_t count = std::min<size_t>(SUM_LIST, ctx->sums.size() - first);
+    int dim = 0;
+    for (size_t i = 0; i < count; ++i) {
+      list.of[i] = ctx->sums[first + i];
+      dim = std::max(dim, list.of[i].dim);
+    }
+    omx_launch(ctx, column_sum_list_kernel, dim3((dim + 63) / 64, static_cast<unsigned>(count)), dim3(1024), 0, list, ctx->fault);
+    OMX_LAUNCH_CHECK(ctx, "column_sum_list_kernel");
+  }
+  ctx->sums.clear();
+  ctx->sums_used = 0;
+  return OMX_OK;
+}
+}  // namespace
+
+// The rows are those of the wide kernel, whose order the list keeps. Full memory is formed and used again. Rows of more than 1 MiB
+// are added at once: 16384 rows of 768 leave 1.5 MiB a norm, and the step that makes 25 of them, whose clock its products hold down,
+// took 18.26 ms with one launch for all where it takes 18.22 with one each.
+float* omx_partial_rows(omx_ctx* ctx, uint64_t blocks, uint64_t dim) {
+  if (!ctx->sums_wait || blocks <= 16 || blocks > OMX_COLUMN_SUM_WIDE_ROWS) return nullptr;
+  constexpr uint64_t kMost = 64ull << 20;
+  const uint64_t bytes = (blocks * dim * sizeof(float) + 255) / 256 * 256;
+  if (bytes > 1ull << 20) return nullptr;
+  if (ctx->sums_used + bytes > ctx->workspace_bytes[kSumsSlot] && form_sums(ctx) != OMX_OK) return nullptr;
+  const uint64_t held = ctx->workspace_bytes[kSumsSlot];
+  uint64_t want = held >= ctx->sums_used + bytes ? held : std::max(bytes, std::min(kMost, bytes * ctx->sums_expected));
+  while (want >= 8 * bytes && !omx_workspace_fits(ctx, want, kSumsSlot)) want /= 2;
+  void* arena = omx_workspace_if_room(ctx, want, kSumsSlot);
+  if (!arena) return nullptr;
+  float* at = reinterpret_cast<float*>(static_cast<char*>(arena) + ctx->sums_used);
+  ctx->sums_used += bytes;
+  return at;
+}
+
 extern "C" {
+
+int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected) {
+  OMX_REQUIRE_CTX(ctx);
+  ctx->sums.clear();
+  ctx->sums_used = 0;
+  ctx->sums_expected = expected;
+  ctx->sums_wait = true;
+  return OMX_OK;
+}
+
+int32_t omx_form_weight_sums(omx_ctx* ctx, int32_t form) {
+  OMX_REQUIRE_CTX(ctx);
+  ctx->sums_wait = false;
+  if (form) return form_sums(ctx);
+  ctx->sums.clear();
+  ctx->sums_used = 0;
+  return OMX_OK;
+}
 
 int32_t omx_rms_norm_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* w, void* y, int32_t y_dtype,
                              uint64_t rows, uint64_t dim, float eps) {

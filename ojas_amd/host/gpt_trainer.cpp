@@ -215,6 +215,20 @@ int32_t forward(ogpt* t) {
   return OMX_OK;
 }
 
+// Weight gradients of the norms wait for one launch (omx_defer_weight_sums); forgotten where the backward ends early.
+struct WaitingSums {
+  omx_ctx* ctx;
+  bool formed = false;
+  WaitingSums(omx_ctx* c, uint32_t count) : ctx(c) { (void)omx_defer_weight_sums(ctx, count); }
+  ~WaitingSums() {
+    if (!formed) (void)omx_form_weight_sums(ctx, 0);
+  }
+  int32_t form() {
+    formed = true;
+    return omx_form_weight_sums(ctx, 1);
+  }
+};
+
 int32_t backward(ogpt* t) {
   omx_ctx* ctx = t->ctx;
   const ogpt_config& c = t->c;
@@ -236,6 +250,7 @@ int32_t backward(ogpt* t) {
   auto slice = [&](void* all, uint64_t l, uint64_t per_layer) {
     return static_cast<void*>(static_cast<char*>(all) + l * per_layer * t->asz);
   };
+  WaitingSums sums(ctx, 2 * c.layers + 1);
   float* gres = keep32 ? static_cast<float*>(slice(t->gyd_all, c.layers - 1, N * d)) : t->gres;
   TRY(omx_rms_norm_backward(ctx, t->x_final, OMX_F32, t->w32(t->nf()), t->ghf, AD, gres, OMX_F32, t->g(t->nf()), N, d,
                             eps));
@@ -297,6 +312,7 @@ int32_t backward(ogpt* t) {
                                        t->g(t->li(l, 0)), N, d, eps));
     gy = AD == OMX_BF16 ? static_cast<const void*>(t->gy16) : static_cast<const void*>(t->gres);
   }
+  TRY(sums.form());
   if (defer) {
     // gw[l](o, j) = sum_r gy[l][r, o] * x[l][r, j] for every layer l in one launch per weight:
     // 4 x layers long reductions with small outputs become four products with enough tiles to fill

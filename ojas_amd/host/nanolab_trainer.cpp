@@ -237,6 +237,21 @@ int32_t forward(onano* t) {
   return OMX_OK;
 }
 
+// Weight gradients of the norms and bias gradients of the gates wait for one launch (omx_defer_weight_sums); forgotten where the
+// backward ends early.
+struct WaitingSums {
+  omx_ctx* ctx;
+  bool formed = false;
+  WaitingSums(omx_ctx* c, uint32_t count) : ctx(c) { (void)omx_defer_weight_sums(ctx, count); }
+  ~WaitingSums() {
+    if (!formed) (void)omx_form_weight_sums(ctx, 0);
+  }
+  int32_t form() {
+    formed = true;
+    return omx_form_weight_sums(ctx, 1);
+  }
+};
+
 int32_t backward(onano* t, float loss_seed) {
   omx_ctx* ctx = t->ctx;
   const onano_config& c = t->c;
@@ -259,6 +274,7 @@ int32_t backward(onano* t, float loss_seed) {
     }
     TRY(omx_scale_grad(ctx, t->g(0), loss_seed, static_cast<uint64_t>(c.vocab) * d));
   }
+  WaitingSums sums(ctx, 3 * c.layers + 1);
   TRY(omx_rms_norm_backward(ctx, t->x_final, OMX_F32, t->w32(t->nf()), t->ghf, AD, t->gres, OMX_F32, t->g(t->nf()), N, d,
                             eps));
   const bool defer = t->deferred_dw;  // implies the bf16 tier
@@ -397,6 +413,7 @@ int32_t backward(onano* t, float loss_seed) {
                                        copy_below, t->g(t->li(l, NORM1)), N, d, eps));
     gy = AD == OMX_BF16 ? static_cast<const void*>(copy_below) : static_cast<const void*>(t->gres);
   }
+  TRY(sums.form());
   if (defer) {
     // gw[l](o, j) = sum_r gy[l][r, o] * x[l][r, j] for every block l, one launch per weight.
     const uint64_t layers = c.layers, per_layer = t->slots[t->li(1, WQ)].offset - t->slots[t->li(0, WQ)].offset;

@@ -714,3 +714,35 @@ def test_a_launch_of_more_threads_than_there_may_be_is_refused(be):
         be.embedding_forward(table, ids)
     assert e.value.code == OUT_OF_RANGE
     assert np.array_equal(be.download(be.residual_add_forward(table, table)), np.full((2, 1), 2.0, np.float32))
+
+
+@pytest.mark.parametrize("count,budget_mib", [(3, 0), (70, 0), (70, 24)])
+def test_weight_sums_that_wait_have_the_same_bits(count, budget_mib):
+    # More than a launch takes, widths that share one, and a budget with room for some of the partial rows.
+    from ojas_amd.backend import F32, MiBackend
+
+    rng = np.random.default_rng(count)
+    be = MiBackend(0, budget_bytes=budget_mib << 20)
+    try:
+        shapes = [(2048 - 13 * i, (256, 512, 260)[i % 3]) for i in range(count)]
+        x = be.upload(rng.normal(0, 1, 2048 * 512).astype(np.float32))
+        gy = be.upload(rng.normal(0, 1, 2048 * 512).astype(np.float32))
+        w = be.upload(rng.normal(1, 0.1, 512).astype(np.float32))
+        gx = be.empty((2048 * 512,), F32)
+
+        def run():
+            grads = be.zeros((count, 512))
+            for i, (rows, dim) in enumerate(shapes):
+                be._check(be._lib.omx_rms_norm_backward(
+                    be._ctx, be._p(x), C.c_int32(F32), be._p(w), be._p(gy), C.c_int32(F32), be._p(gx), C.c_int32(F32),
+                    C.c_void_p(grads.ptr + i * 2048), C.c_uint64(rows), C.c_uint64(dim), C.c_float(1e-6)))
+            return grads
+
+        want = be.download(run())
+        be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(count)))
+        waiting = run()
+        be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
+        assert np.array_equal(be.download(waiting), want)
+        assert np.array_equal(be.download(run()), want)  # formed at once again
+    finally:
+        be.close()
