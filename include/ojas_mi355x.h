@@ -448,6 +448,10 @@ int32_t omx_muon_ns5_step_batched(omx_ctx* ctx, void* const* params_f32, const v
 int32_t omx_muon_ns5_step_list(omx_ctx* ctx, void* const* params_f32, const void* const* grads_f32,
                                void* const* momenta_f32, void* const* params_bf16, uint64_t count,
                                uint64_t rows, uint64_t cols, const omx_muon_config* config);
+/* omx_muon_ns5_step_list over tensors of any shapes (rows[i] x cols[i]): the products of small f32 shapes go out together. */
+int32_t omx_muon_ns5_step_shapes(omx_ctx* ctx, void* const* params_f32, const void* const* grads_f32,
+                                 void* const* momenta_f32, void* const* params_bf16, const uint64_t* rows,
+                                 const uint64_t* cols, uint64_t count, const omx_muon_config* config);
 /* Bytes of device scratch omx_muon_ns5_step takes from the budget
  * (BackendCore::optimizer_scratch_bytes, backend.rs:938-961). */
 uint64_t omx_muon_scratch_bytes(uint64_t rows, uint64_t cols);

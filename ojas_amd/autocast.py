@@ -178,3 +178,8 @@ class Autocast:
         self.inner.muon_ns5_step_list(params, grads, momenta, *args, **kwargs)
         for t in (*params, *momenta):
             self._wrote(t)
+
+    def muon_ns5_step_shapes(self, params, grads, momenta, *args, **kwargs):
+        self.inner.muon_ns5_step_shapes(params, grads, momenta, *args, **kwargs)
+        for t in (*params, *momenta):
+            self._wrote(t)

@@ -647,6 +647,16 @@ class MiBackend(_native.Methods):
         self._check_lists("muon_ns5_step", shapes.muon_ns5_step_dims, (params, grads, momenta), rank=2)
         self._muon_list(_native.omx_muon_ns5_step_list, params, grads, momenta, config, params_bf16)
 
+    def muon_ns5_step_shapes(self, params, grads, momenta, config: MuonNs5Config, params_bf16=None):
+        """`muon_ns5_step_list` over matrices of any shapes: the products of small shapes go out together."""
+        self._check_lists("muon_ns5_step", shapes.muon_ns5_step_dims, (params, grads, momenta), rank=2)
+        n = len(params)
+        table = lambda ts: (C.c_void_p * n)(*[(t.ptr if t is not None else None) for t in ts])
+        extent = lambda axis: (C.c_uint64 * n)(*[t.shape[axis] for t in params])
+        tables = [table(params), table(grads), table(momenta), table(params_bf16) if params_bf16 else None, extent(0), extent(1)]
+        _native.omx_muon_ns5_step_shapes(self._context, *[C.addressof(t) if t is not None else None for t in tables], n,
+                                         C.addressof(config))
+
     def _muon_list(self, entry, params, grads, momenta, config, params_bf16):
         n = len(params)
         rows, cols = params[0].shape

@@ -340,6 +340,21 @@ int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);
 constexpr int FRAG32_TILES = 5, DMA32_TILES = 4;
 double omx_gemm_frag32_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
 int32_t omx_gemm_frag32_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
+// Independent f32 products C = A.B, or s1 aux + s2 A.B where `aux` is set (C's layout), in one launch; strides in elements, as
+// omx_gemm_impl's; `stride`: between the `batches` products of a strided batch, of every operand. `symmetric`: every C equals its
+// transpose.
+struct OmxGemmProduct {
+  const float* a;
+  uint64_t a_rs, a_cs;
+  const float* b;
+  uint64_t b_rs, b_cs;
+  float* c;
+  uint64_t ldc, m, k, n;
+  const float* aux;
+  uint64_t batches, stride;
+};
+constexpr int FRAG32_GROUP = 8;
+int32_t omx_gemm_frag32_group(omx_ctx* ctx, const OmxGemmProduct* products, int count, bool symmetric, float s1, float s2, unsigned long long tag);
 bool omx_gemm_dma32_eligible(const GemmArgs& g, bool a_km, bool b_km);
 double omx_gemm_dma32_us(omx_ctx* ctx, const GemmArgs& g, int tile);
 void omx_gemm_dma32_tile(int tile, int* bm, int* bn);

@@ -88,33 +88,61 @@ struct Frag32 {
   }
 };
 
-template <bool A_KM, bool B_KM, int MB, int NB, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
-  constexpr int BM = 16 * MB, BN = 16 * NB, PITCH32 = BN + 4;  // the pad keeps 16-byte pieces and spreads banks
-  extern __shared__ __attribute__((aligned(16))) float sums[];  // [WAVES][BM][PITCH32]
-  const int total = g.tiles_m * g.tiles_n, r = tile_of_eighth(blockIdx.x, total * g.batches);
-  const int product = r / total, id = r - product * total;
-  // An XCD's run of tiles spans the output's shorter side.
-  const int tile_m = g.tiles_m >= g.tiles_n ? id / g.tiles_n : id % g.tiles_m;
-  const int tile_n = g.tiles_m >= g.tiles_n ? id % g.tiles_n : id / g.tiles_m;
-  gemm_select_batch(g, product);
+// A wave's share of a tile's sums into its part of [WAVES][16 MB][16 NB + 4] in LDS. acc[m][n][v]: A's row i = lane % 16 of block
+// m, B's row 4 (lane / 16) + v of block n.
+template <bool A_KM, bool B_KM, int MB, int NB>
+__device__ __forceinline__ void frag32_share(const floatx4_f (&acc)[MB][NB], int lane, int wave, float* sums) {
+  constexpr int BM = 16 * MB, PITCH32 = 16 * NB + 4;
+  float* mine = sums + wave * (BM * PITCH32);
+  const int i = lane & 15, kg = lane >> 4;
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    float* r = mine + (A_KM ? MB * i + m : 16 * m + i) * PITCH32;
+    if constexpr (!B_KM) {
+#pragma unroll
+      for (int n = 0; n < NB; ++n) *reinterpret_cast<floatx4_f*>(r + 16 * n + 4 * kg) = acc[m][n];
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) r[NB * (4 * kg + v) + n] = acc[m][n][v];
+    }
+  }
+}
+
+// The waves' shares of a tile. FOLD: every step of 16 K values sums into registers of its own that are added to the wave's total
+// when the next one starts, chains of 16 and of K / (16 WAVES) instead of one of K / WAVES.
+template <bool A_KM, bool B_KM, int MB, int NB, int WAVES, bool FOLD>
+__device__ __forceinline__ void frag32_sums(const GemmArgs& g, int row0, int col0, float* sums) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int row0 = tile_m * BM, col0 = tile_n * BN;
   Frag32<A_KM, MB> fa;
   Frag32<B_KM, NB> fb;
   fa.init(static_cast<const float*>(g.a), g.lda, row0, g.M, lane);
   fb.init(static_cast<const float*>(g.b), g.ldb, col0, g.N, lane);
-  floatx4_f acc[MB][NB];
+  floatx4_f acc[MB][NB], step_sum[MB][NB];
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int n = 0; n < NB; ++n) acc[m][n] = floatx4_f{0.0f, 0.0f, 0.0f, 0.0f};
-  auto multiply = [&](const float (&a)[MB][4], const float (&b)[NB][4], int j) {
+    for (int n = 0; n < NB; ++n) acc[m][n] = step_sum[m][n] = floatx4_f{0.0f, 0.0f, 0.0f, 0.0f};
+  auto fold = [&]() {
 #pragma unroll
     for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int n = 0; n < NB; ++n)
-        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[n][j], a[m][j], acc[m][n], 0, 0, 0);
+      for (int n = 0; n < NB; ++n) acc[m][n] += step_sum[m][n];
+  };
+  auto multiply = [&](const float (&a)[MB][4], const float (&b)[NB][4], int j) {
+    if (FOLD && j == 0) fold();
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        if constexpr (FOLD) {
+          const floatx4_f c = j == 0 ? floatx4_f{0.0f, 0.0f, 0.0f, 0.0f} : step_sum[m][n];
+          step_sum[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[n][j], a[m][j], c, 0, 0, 0);
+        } else {
+          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[n][j], a[m][j], acc[m][n], 0, 0, 0);
+        }
+      }
   };
   // Sets of fragments: one in use, two on their way. A quarter of a step's loads follows each quarter of its products: all
   // of them at once hold up the products behind them (loads between 64 and 128 products in a row: 97 and 133 us for 8192 x
@@ -159,22 +187,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) multiply(a[0], b[0], j);
   }
-  // acc[m][n][v]: A's row i = lane % 16 of block m, B's row 4 (lane / 16) + v of block n, this wave's share of K.
-  float* mine = sums + wave * (BM * PITCH32);
-  const int i = lane & 15, kg = lane >> 4;
-#pragma unroll
-  for (int m = 0; m < MB; ++m) {
-    float* r = mine + (A_KM ? MB * i + m : 16 * m + i) * PITCH32;
-    if constexpr (!B_KM) {
-#pragma unroll
-      for (int n = 0; n < NB; ++n) *reinterpret_cast<floatx4_f*>(r + 16 * n + 4 * kg) = acc[m][n];
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-#pragma unroll
-        for (int n = 0; n < NB; ++n) r[NB * (4 * kg + v) + n] = acc[m][n][v];
-    }
-  }
+  if constexpr (FOLD) fold();
+  frag32_share<A_KM, B_KM>(acc, lane, wave, sums);
+}
+
+template <bool A_KM, bool B_KM, int MB, int NB, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
+  constexpr int BM = 16 * MB, BN = 16 * NB, PITCH32 = BN + 4;  // the pad keeps 16-byte pieces and spreads banks
+  extern __shared__ __attribute__((aligned(16))) float sums[];  // [WAVES][BM][PITCH32]
+  const int total = g.tiles_m * g.tiles_n, r = tile_of_eighth(blockIdx.x, total * g.batches);
+  const int product = r / total, id = r - product * total;
+  // An XCD's run of tiles spans the output's shorter side.
+  const int tile_m = g.tiles_m >= g.tiles_n ? id / g.tiles_n : id % g.tiles_m;
+  const int tile_n = g.tiles_m >= g.tiles_n ? id % g.tiles_n : id / g.tiles_m;
+  gemm_select_batch(g, product);
+  const int row0 = tile_m * BM, col0 = tile_n * BN;
+  frag32_sums<A_KM, B_KM, MB, NB, WAVES, false>(g, row0, col0, sums);
   __syncthreads();
   bool bad = false;
   for (int c = threadIdx.x; c < BM * (BN / 4); c += WAVES * 64) {
@@ -188,6 +216,83 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
     if (row0 + r < g.M && col0 + cc < g.N) bad |= gemm_store4(g, 0, row0 + r, col0 + cc, t.x, t.y, t.z, t.w);
   }
   if (bad) dev_raise_fault(g.fault, g.tag);
+}
+
+// ---- several products in one launch ----
+// Five shapes of a model's matrices are five chains of fifteen Newton-Schulz products, each a launch of 4 to 256 workgroups that takes
+// 3 to 13 us and leaves most of the chip idle: the k-th products of all chains go out together. 32 x 32 tiles whose four waves share
+// K. Four blocks of d = 256 (32 matrices): 33, 26 and 40 us for the first, second and third products of an iteration, 20, 13 and 28
+// in one launch each; bound by the waits of short walks over K (a third of the f32 matrix rate). 64 x 32 tiles took 22, 16 and 30,
+// steps of 32 K values with all of a step's loads together 28, 16 and 33.
+// `symmetric`: the output equals its transpose (X X^T, A A and their sums with a symmetric tensor): tiles below the diagonal are
+// written from those above it, the same sums in the same order.
+constexpr int GROUP_WAVES = 4, GROUP_TILE = 32;
+struct FragProduct {
+  const float *a, *b, *aux;
+  float* c;
+  long lda, ldb, ldc, batch;  // batch: BYTES between the products of a strided batch, in every operand
+  int M, N, K, tiles_m, tiles_n, batches, layout, c_vec;  // layout: 2 A k-major + B k-major
+};
+struct FragGroup {
+  FragProduct product[FRAG32_GROUP];
+  int first[FRAG32_GROUP];  // a product's first workgroup, a multiple of 8
+  int symmetric;
+  float s1, s2;
+  OmxFaultWord* fault;
+  unsigned long long tag;
+};
+__global__ __launch_bounds__(GROUP_WAVES * 64) void gemm_frag32_group_kernel(FragGroup q) {
+  __shared__ __align__(16) float sums[GROUP_WAVES * GROUP_TILE * (GROUP_TILE + 4)];
+  constexpr int PITCH32 = GROUP_TILE + 4;
+  int which = 0;  // (all of `first` in one load)
+#pragma unroll
+  for (int i = 1; i < FRAG32_GROUP; ++i) which += static_cast<int>(blockIdx.x) >= q.first[i];
+  const FragProduct& p = q.product[which];
+  const int total = p.tiles_m * p.tiles_n, index = blockIdx.x - q.first[which];
+  if (index >= total * p.batches) return;
+  const int r = tile_of_eighth(index, total * p.batches), product = r / total, id = r - product * total;
+  const int tile_m = id / p.tiles_n, tile_n = id - tile_m * p.tiles_n;
+  if (q.symmetric && tile_m > tile_n) return;
+  GemmArgs g;
+  const long shift = product * p.batch;
+  g.a = reinterpret_cast<const char*>(p.a) + shift;
+  g.b = reinterpret_cast<const char*>(p.b) + shift;
+  g.c = reinterpret_cast<char*>(p.c) + shift;
+  g.aux_in = p.aux ? reinterpret_cast<const unsigned short*>(reinterpret_cast<const char*>(p.aux) + shift) : nullptr;
+  g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc;
+  g.M = p.M; g.N = p.N; g.K = p.K;
+  g.c_bf16 = 0;
+  g.accumulate = p.aux ? 2 : 0;
+  g.c_vec = p.c_vec;
+  g.splits = 1;
+  g.epi_s1 = q.s1; g.epi_s2 = q.s2;
+  const int row0 = tile_m * GROUP_TILE, col0 = tile_n * GROUP_TILE;
+  switch (p.layout) {  // (uniform)
+    case 0: frag32_sums<false, false, 2, 2, GROUP_WAVES, true>(g, row0, col0, sums); break;
+    case 1: frag32_sums<false, true, 2, 2, GROUP_WAVES, true>(g, row0, col0, sums); break;
+    case 2: frag32_sums<true, false, 2, 2, GROUP_WAVES, true>(g, row0, col0, sums); break;
+    default: frag32_sums<true, true, 2, 2, GROUP_WAVES, true>(g, row0, col0, sums);
+  }
+  __syncthreads();
+  // 256 threads, 256 pieces of four columns.
+  const int row = threadIdx.x / (GROUP_TILE / 4), col = threadIdx.x % (GROUP_TILE / 4) * 4;
+  auto meet = [&](int at, int step, float (&t)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = sums[at + e * step];
+#pragma unroll
+    for (int w = 1; w < GROUP_WAVES; ++w)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) t[e] += sums[w * (GROUP_TILE * PITCH32) + at + e * step];
+  };
+  bool bad = false;
+  float t[4];
+  meet(row * PITCH32 + col, 1, t);
+  if (row0 + row < g.M && col0 + col < g.N) bad |= gemm_store4(g, 0, row0 + row, col0 + col, t[0], t[1], t[2], t[3]);
+  if (q.symmetric && tile_m != tile_n) {
+    meet(col * PITCH32 + row, PITCH32, t);
+    if (col0 + row < g.M && row0 + col < g.N) bad |= gemm_store4(g, 0, col0 + row, row0 + col, t[0], t[1], t[2], t[3]);
+  }
+  if (bad) dev_raise_fault(q.fault, q.tag);
 }
 
 struct FragTile {
@@ -252,4 +357,50 @@ int32_t omx_gemm_frag32_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool 
   if (!a_km) return launch_frag_tile<false, true>(ctx, g, tile);
   if (!b_km) return launch_frag_tile<true, false>(ctx, g, tile);
   return launch_frag_tile<true, true>(ctx, g, tile);
+}
+
+// (The operands are the library's own scratch: what does not fit is a mistake of the caller's.)
+static bool group_fits(const OmxGemmProduct& p) {
+  const bool a_km = p.a_cs != 1, b_km = p.b_rs != 1;
+  const long lda = static_cast<long>(a_km ? p.a_cs : p.a_rs), ldb = static_cast<long>(b_km ? p.b_rs : p.b_cs);
+  const uint64_t most = 0x7fffffff, tiles = (p.m + GROUP_TILE - 1) / GROUP_TILE * ((p.n + GROUP_TILE - 1) / GROUP_TILE);
+  return p.m <= most && p.n <= most && p.k <= most && p.batches > 0 && tiles <= most / FRAG32_GROUP / p.batches - 8 && p.stride % 4 == 0 &&
+         (!a_km || p.a_rs == 1) && (!b_km || p.b_cs == 1) &&
+         frag_fits(a_km, p.a, lda, static_cast<int>(p.m), 2, 0) && frag_fits(b_km, p.b, ldb, static_cast<int>(p.n), 2, 0);
+}
+
+int32_t omx_gemm_frag32_group(omx_ctx* ctx, const OmxGemmProduct* products, int count, bool symmetric, float s1, float s2, unsigned long long tag) {
+  FragGroup q;
+  q.symmetric = symmetric;
+  q.s1 = s1;
+  q.s2 = s2;
+  q.fault = ctx->fault;
+  q.tag = tag;
+  int at = 0;
+  for (int i = 0; i < count; ++i) {
+    const OmxGemmProduct& p = products[i];
+    if (!group_fits(p)) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: products in one launch", omx_fault_name(tag & 0x7f));
+    FragProduct& f = q.product[i];
+    const bool a_km = p.a_cs != 1, b_km = p.b_rs != 1;
+    f.a = p.a; f.b = p.b; f.aux = p.aux; f.c = p.c;
+    f.lda = static_cast<long>(a_km ? p.a_cs : p.a_rs);
+    f.ldb = static_cast<long>(b_km ? p.b_rs : p.b_cs);
+    f.ldc = static_cast<long>(p.ldc);
+    f.batch = static_cast<long>(p.stride) * 4;
+    f.M = static_cast<int>(p.m); f.N = static_cast<int>(p.n); f.K = static_cast<int>(p.k);
+    f.tiles_m = (f.M + GROUP_TILE - 1) / GROUP_TILE;
+    f.tiles_n = (f.N + GROUP_TILE - 1) / GROUP_TILE;
+    f.batches = static_cast<int>(p.batches);
+    f.layout = 2 * a_km + b_km;
+    f.c_vec = (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0 && p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.aux) & 15u) == 0;
+    q.first[i] = at;
+    at += (f.tiles_m * f.tiles_n * f.batches + 7) & ~7;
+  }
+  for (int i = count; i < FRAG32_GROUP; ++i) {
+    q.first[i] = 0x7fffffff;
+    q.product[i] = FragProduct{};
+  }
+  omx_launch(ctx, gemm_frag32_group_kernel, dim3(static_cast<unsigned>(at)), dim3(GROUP_WAVES * 64), 0, q);
+  OMX_LAUNCH_CHECK(ctx, "gemm_frag32_group_kernel");
+  return OMX_OK;
 }

@@ -306,12 +306,14 @@ class NanolabTrainer:
                 be.scale_grad(loss, weight)
             loss_sum = loss if loss_sum is None else be.residual_add_forward(loss_sum, loss)
         grad_norm = be.clip_grad_norm([acc[n] for n in self.trainable], self.grad_clip)
-        # One set of launches for the matrices of each shape, one for everything AdamW steps: a tensor at a time, a small
+        # One set of launches for the matrices of all shapes, one for everything AdamW steps: a tensor at a time, a small
         # model's 32 matrices took 990 launches and its 25 vectors 75, most of the step's time.
         cfg = MuonNs5Config(self.matrix_lr * lr_multiplier, MUON_MOMENTUM, MUON_WEIGHT_DECAY, 1, int(self.ns5_bf16))
-        for names in self.muon_groups:
-            be.muon_ns5_step_list([self.params[n] for n in names], [acc[n] for n in names],
-                                  [self.state[n][0] for n in names], cfg)
+        # (A subclass or wrapper of the backend, which may count, tag or check calls, gets one for each shape.)
+        together = type(be.inner if self.autocast else be) is MiBackend
+        for names in [sum(self.muon_groups, [])] if together and self.muon_groups else self.muon_groups:
+            step = be.muon_ns5_step_shapes if together else be.muon_ns5_step_list
+            step([self.params[n] for n in names], [acc[n] for n in names], [self.state[n][0] for n in names], cfg)
         cfg = AdamWConfig.nanolab(self.adam_lr * lr_multiplier, ADAM_HYBRID_WEIGHT_DECAY)
         be.adamw_step_batched([self.params[n] for n in self.adam], [acc[n] for n in self.adam],
                               [self.state[n][0] for n in self.adam], [self.state[n][1] for n in self.adam], self.step, cfg)

@@ -281,3 +281,99 @@ def test_f32_iteration_sums_in_the_store_pass_carry_the_separate_kernels_bits(be
     for a, b in zip(got[1], got[0]):
         assert np.array_equal(a, b)
     assert any(np.any(a != p) for a, p in zip(got[1][:count], ps))
+
+
+# (rows, cols, tensors) of a call; widths off the 32 x 32 tile and off the 16-column step of K, more shapes than a launch takes products
+# of, more tensors than a launch takes, and shapes that keep their own launches (130 x 70).
+MIXES = [
+    [(256, 256, 3), (128, 256, 2), (4, 256, 2), (704, 256, 2), (256, 704, 1)],
+    [(64, 48, 2), (36, 100, 1), (100, 36, 1), (130, 70, 2), (4, 4, 1), (4, 32, 1), (32, 4, 1), (12, 20, 1), (8, 72, 1), (60, 60, 1), (68, 44, 1)],
+    [(32, 32, 50), (32, 64, 30)],
+]
+
+
+@pytest.mark.parametrize("mix", MIXES)
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_shapes_step_matches_the_oracle_per_tensor(be, mix, bf16):
+    """`muon_ns5_step_shapes` at the single op's gates (momentum bit for bit; update 2e-3 of its largest element in f32,
+    5e-2 with the bf16 iteration), tensors of one shape apart from each other in the call."""
+    from ojas_amd.backend import BF16, MuonNs5Config
+
+    print(f"muon shapes {mix} bf16={bf16}", flush=True)
+    r = np.random.default_rng(len(mix))
+    dims = [(rows, cols) for rows, cols, n in mix for _ in range(n)]
+    dims = [dims[i] for i in r.permutation(len(dims))]
+    ps, gs, ms = ([(r.standard_normal(d) * size).astype(np.float32) for d in dims] for size in (0.1, 0.05, 0.01))
+    cfg = MuonNs5Config(0.02, 0.95, 0.1, 1, bf16)
+    dp, dg, dm = [be.upload(x) for x in ps], [be.upload(x) for x in gs], [be.upload(x) for x in ms]
+    mirrors = [be.upload(np.zeros(d, np.float32), BF16) if i % 2 == 0 else None for i, d in enumerate(dims)]
+    be.muon_ns5_step_shapes(dp, dg, dm, cfg, mirrors)
+    be.sync()
+    orc.set_threads(8)
+    decay = np.float32(1.0 - 0.02 * 0.1)
+    for i in range(len(dims)):
+        op, om = orc.muon_ns5_step(ps[i], gs[i], ms[i], lr=0.02, momentum=0.95, weight_decay=0.1, nesterov=True, bf16=bool(bf16))
+        assert np.array_equal(be.download(dm[i]), om), dims[i]
+        got = be.download(dp[i])
+        upd_gpu, upd_cpu = got - ps[i] * decay, op - ps[i] * decay
+        assert np.max(np.abs(upd_gpu - upd_cpu)) <= (5e-2 if bf16 else 2e-3) * np.max(np.abs(upd_cpu)), dims[i]
+        if mirrors[i] is not None:
+            assert np.array_equal(be.download(mirrors[i]), orc.to_bf16(got)), dims[i]
+
+
+def test_shapes_step_refuses_each_matrix_by_itself(be):
+    """As the list's test, across shapes; and a configuration or a shape that is refused steps nothing."""
+    from ojas_amd.backend import NON_FINITE, OUT_OF_RANGE, SHAPE, MuonNs5Config, OjasError
+
+    print("muon shapes refusals", flush=True)
+    r = np.random.default_rng(8)
+    dims = [(64, 48), (32, 96), (64, 48), (130, 70), (96, 32), (32, 96)]
+    ps, gs, ms = ([(r.standard_normal(d) * s).astype(np.float32) for d in dims] for s in (0.1, 0.05, 0.01))
+    bad_g, bad_m = [g.copy() for g in gs], [m.copy() for m in ms]
+    bad_g[0][3, 5] = np.nan
+    bad_m[3][-1, -1] = np.inf
+    bad_g[5][:] = 3e38
+    cfg = MuonNs5Config(0.02, 0.95, 0.1, 1, 0)
+    out = []
+    for g, m in ((gs, ms), (bad_g, bad_m)):
+        dp, dg, dm = [be.upload(x) for x in ps], [be.upload(x) for x in g], [be.upload(x) for x in m]
+        be.muon_ns5_step_shapes(dp, dg, dm, cfg)
+        if g is bad_g:
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.code == NON_FINITE and "muon_ns5_step" in str(e.value)
+        out.append([(be.download(p), be.download(m)) for p, m in zip(dp, dm)])
+    for i in range(6):
+        if i in (0, 3, 5):
+            assert np.array_equal(out[1][i][0], ps[i]) and np.array_equal(out[1][i][1], bad_m[i]), i
+        else:
+            assert np.array_equal(out[1][i][0], out[0][i][0]) and np.array_equal(out[1][i][1], out[0][i][1]), i
+    dp, dg, dm = [be.upload(x) for x in ps], [be.upload(x) for x in gs], [be.upload(x) for x in ms]
+    with pytest.raises(OjasError) as e:
+        be.muon_ns5_step_shapes(dp, dg, dm, MuonNs5Config(-0.1, 0.9, 0.0, 1, 0))
+    assert e.value.code == OUT_OF_RANGE
+    with pytest.raises(OjasError) as e:
+        be.muon_ns5_step_shapes(dp, [dg[1]] + dg[1:], dm, cfg)
+    assert e.value.code == SHAPE
+    be.sync()
+    assert all(np.array_equal(be.download(d), p) for d, p in zip(dp + dm, ps + ms))
+
+
+def test_shapes_step_takes_the_scratch_there_is():
+    """Room for the scratch of the largest two tensors of seven: two or three at a time, each held to the oracle."""
+    from ojas_amd.backend import MiBackend, MuonNs5Config
+
+    print("muon shapes under a budget", flush=True)
+    r = np.random.default_rng(3)
+    dims = [(256, 512), (256, 256), (256, 512), (256, 256), (512, 256), (128, 512), (256, 256)]
+    ps, gs, ms = ([(r.standard_normal(d) * s).astype(np.float32) for d in dims] for s in (0.1, 0.05, 0.01))
+    small = MiBackend(0, budget_bytes=3 * 4 * sum(a * b for a, b in dims) + (6 << 20))
+    dp, dg, dm = [small.upload(x) for x in ps], [small.upload(x) for x in gs], [small.upload(x) for x in ms]
+    small.muon_ns5_step_shapes(dp, dg, dm, MuonNs5Config(0.02, 0.95, 0.1, 1, 0))
+    decay = np.float32(1.0 - 0.02 * 0.1)
+    for i in range(len(dims)):
+        op, om = orc.muon_ns5_step(ps[i], gs[i], ms[i], lr=0.02, momentum=0.95, weight_decay=0.1, nesterov=True, bf16=False)
+        assert np.array_equal(small.download(dm[i]), om), i
+        upd_gpu, upd_cpu = small.download(dp[i]) - ps[i] * decay, op - ps[i] * decay
+        assert np.max(np.abs(upd_gpu - upd_cpu)) <= 2e-3 * np.max(np.abs(upd_cpu)), i
+    small.close()
