@@ -1249,8 +1249,13 @@ bool at_prompt(const Sdpa32Args& a, int dim, bool bf16_cache) {
 
 // Rows per workgroup of the forward.
 long forward_rows(omx_ctx* ctx, const Sdpa32Args& a, int dim, long planes, long rows, bool bf16_cache) {
-  if (at_prompt(a, dim, bf16_cache))  // Twice the rows on a key's way only where half as many workgroups still fill the chip.
-    return dim == 64 && (rows + 31) / 32 * planes >= 4l * (ctx->cu_count > 0 ? ctx->cu_count : 256) ? 32 : 16;
+  if (at_prompt(a, dim, bf16_cache)) {
+    // Twice the rows on a key's way where the chip has a workgroup of them for every unit and the fullest unit has less to do: one
+    // takes 1.6 to 1.9 times as long as one of 16 rows. Workgroups of 16 rows, us with 16 / 32 rows: 512 17.0 / 13.9, 768 17.3 / 18.6,
+    // 1024 17.8 / 15.2, 1152 24.4 / 24.2, 1536 35.2 / 32.8.
+    const long units = ctx->cu_count > 0 ? ctx->cu_count : 256, few = (rows + 31) / 32 * planes, many = (rows + 15) / 16 * planes;
+    return dim == 64 && few >= units && 7 * ((few + units - 1) / units) < 4 * ((many + units - 1) / units) ? 32 : 16;
+  }
   return at_narrow(ctx, a, planes, rows, at_span(a)) ? 16 : 64;
 }
 
@@ -1260,7 +1265,7 @@ int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) 
   const dim3 grid(static_cast<unsigned>((rows + per - 1) / per), planes, static_cast<unsigned>(std::max(1, a.nparts)));
   if constexpr (D >= 64) {
     if (at_prompt(a, D, bf16_cache)) {  // (attention over a cache has no lse)
-      const bool two = per == 32, split = a.nparts > 1;  // (two: four workgroups per compute unit and more, never split)
+      const bool two = per == 32, split = a.nparts > 1;  // (two: a workgroup per compute unit and more, never split)
       if constexpr (D == 64) {
         if (two) omx_launch(ctx, (sdpa_prompt_kernel<D, 2, false>), grid, dim3(AT_THREADS), 0, a);
       }
@@ -1346,7 +1351,7 @@ int omx_sdpa32_key_parts(omx_ctx* ctx, const Sdpa32Args& a, int batch, int dim, 
   const long keys = prompt ? 4 * (4096 / dim) : AT_ROWS;
   const double step = prompt ? (dim == 64 ? 2.0 : 1.45) : 0.5 + 0.0175 * dim;
   const long steps = (a.tk + keys - 1) / keys, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  const long most = std::min(std::min(2 * cus / blocks, steps), 64l);
+  const long most = per == 32 ? 1 : std::min(std::min(2 * cus / blocks, steps), 64l);  // (32 rows: no form for parts)
   long best = 1;
   double least = 0.0;
   for (long p = 1; p <= std::max(1l, most); ++p) {

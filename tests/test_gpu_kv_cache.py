@@ -256,6 +256,15 @@ def test_prompt_chunks_over_bf16_caches_lose_nothing(be, b, tq, h, hkv, d, capac
 
 
 @pytest.mark.parametrize("b,tq,h,hkv,d,capacity,kv_len,window", [
+    (4, 253, 8, 8, 64, 2100, 2100, None), (2, 128, 64, 32, 64, 1000, 1700, 300), (17, 160, 3, 3, 64, 400, 400, None),
+    (8, 125, 10, 10, 64, 130, 129, None)])
+def test_prompt_blocks_of_32_rows_where_each_unit_has_one(be, b, tq, h, hkv, d, capacity, kv_len, window):
+    """The rule for two blocks of 16 rows per workgroup at its edges: 256 workgroups over keys that a smaller call would
+    part, ring and window, 255, and 320 that do not pay; as above."""
+    test_prompt_chunks_over_bf16_caches_lose_nothing(be, b, tq, h, hkv, d, capacity, kv_len, window)
+
+
+@pytest.mark.parametrize("b,tq,h,hkv,d,capacity,kv_len,window", [
     (1, 17, 2, 2, 64, 320, 320, None), (1, 64, 4, 2, 64, 300, 700, 200), (1, 40, 2, 2, 128, 150, 411, 110), (1, 33, 3, 3, 64, 200, 197, 130),
     (32, 40, 16, 16, 64, 257, 250, None), (1, 24, 2, 1, 128, 129, 129, 97)])
 def test_prompt_tiles_that_every_row_sees(be, b, tq, h, hkv, d, capacity, kv_len, window):
