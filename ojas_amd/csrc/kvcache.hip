@@ -264,7 +264,8 @@ __device__ __forceinline__ float across_groups(float v, F f) {
 template <typename T>
 struct KvPiece {
   float4 q;
-  __device__ __forceinline__ void load(const T* p) { q = *reinterpret_cast<const float4*>(p); }
+  template <bool STREAM>
+  __device__ __forceinline__ void load(const T* p) { q = dev_stream_load<STREAM>(reinterpret_cast<const float4*>(p)); }
   template <bool HOLD>
   __device__ __forceinline__ void get(float (&v)[4]) {
     if constexpr (HOLD) asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(q.z), "+v"(q.w));
@@ -274,7 +275,8 @@ struct KvPiece {
 template <>
 struct KvPiece<unsigned short> {
   uint2 q;
-  __device__ __forceinline__ void load(const unsigned short* p) { q = *reinterpret_cast<const uint2*>(p); }
+  template <bool STREAM>
+  __device__ __forceinline__ void load(const unsigned short* p) { q = dev_stream_load<STREAM>(reinterpret_cast<const uint2*>(p)); }
   template <bool HOLD>
   __device__ __forceinline__ void get(float (&v)[4]) {
     if constexpr (HOLD) asm volatile("" : "+v"(q.x), "+v"(q.y));
@@ -290,7 +292,7 @@ struct KvPiece<unsigned short> {
 // takes more waves of fewer rounds (KG_FEW_WAVES): 15.0 -> 5.3 KiB, 12 heads x 301 positions 12.1 -> 6.5 us.
 // WAVES waves share a block's keys (a contiguous run each) and add up in LDS in wave order. When one block
 // covers a row's whole span (nparts == 1) it writes the output itself: no partials in memory, no second launch.
-template <typename T, int LPK, int WAVES, int ROWS, int ROUNDS>
+template <typename T, int LPK, int WAVES, int ROWS, int ROUNDS, bool STREAM = false>
 __global__ __launch_bounds__(WAVES * 64) void cached_attention_group_kernel(KvArgs a) {
   __shared__ float meet[WAVES][ROWS][LPK * 4 + 2];
   constexpr int G = 64 / LPK;               // keys per round
@@ -361,8 +363,8 @@ __global__ __launch_bounds__(WAVES * 64) void cached_attention_group_kernel(KvAr
       unsigned int slot = slot0 + key;  // a tile wraps the ring at most once
       slot = slot >= capacity ? slot - capacity : slot;
       const size_t off = static_cast<size_t>(((base_b + slot) * a.kv_heads + kvh) * dim + d0);
-      kr[i].load(kc + off);
-      vr[i].load(vc + off);
+      kr[i].template load<STREAM>(kc + off);
+      vr[i].template load<STREAM>(vc + off);
     }
     // Every load goes out before the first product (the compiler otherwise moves products up between them, each with
     // its wait: 64 sequences of 1024 positions, 103 us instead of 73). Four rows have no registers to hold them all.
@@ -623,12 +625,20 @@ int32_t launch_kv_write(omx_ctx* ctx, const KvWrite& w) {
   return OMX_OK;
 }
 
+// Bytes of keys and values from which a call reads them past the caches: half of the memory-side cache, of which a model of two layers
+// and more leaves nothing for the next token. 12 layers, us a call, without and with the hint: 64 x 12 heads x 1024 f32 positions (403 MB)
+// 73.1, 66.4; bf16 (201 MB) 47.3, 45.2; two layers of 118 MB, which stay in the cache, 23.1 and 25.0.
+constexpr uint64_t KV_STREAM = 128ull << 20;
 template <typename T, int LPK, int NPL>
 int32_t launch_group(omx_ctx* ctx, const KvArgs& a, dim3 grid, long rows_total, int waves) {
   auto go = [&](auto most, auto four, auto one) {
     omx_launch(ctx, (waves >= 8 ? most : waves == 4 ? four : one), grid, dim3(waves * 64), 0, a);
   };
-  if (a.tq * a.group == 1)
+  const uint64_t span = std::min<uint64_t>(a.kv_len - a.read_lo, a.capacity);
+  if (a.tq * a.group == 1 && waves <= 4 && 2 * sizeof(T) * a.batch * span * a.kv_heads * a.dim >= KV_STREAM)
+    omx_launch(ctx, (waves == 4 ? &cached_attention_group_kernel<T, LPK, 4, 1, KG_ROUNDS, true> : &cached_attention_group_kernel<T, LPK, 1, 1, KG_ROUNDS, true>),
+               grid, dim3(waves * 64), 0, a);
+  else if (a.tq * a.group == 1)
     go(&cached_attention_group_kernel<T, LPK, KG_FEW_WAVES<T>, 1, 8 * KG_ROUNDS / KG_FEW_WAVES<T>>, &cached_attention_group_kernel<T, LPK, 4, 1, KG_ROUNDS>,
        &cached_attention_group_kernel<T, LPK, 1, 1, KG_ROUNDS>);
   else

@@ -289,7 +289,9 @@ __device__ __forceinline__ float fused_block_sum(float v, float* red) {
   for (int i = 1; i < CE_FUSED_THREADS / 64; ++i) r += red[i];
   return r;
 }
-template <typename T, int MAXV>
+// Bytes of a logits tile from which it is read and its gradient written past the caches (16384 x 50304 bf16: 617 -> 574 us).
+constexpr uint64_t CE_STREAM = 384ull << 20;
+template <typename T, int MAXV, bool STREAM>
 __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __restrict__ tile, size_t ld, size_t row0,
                                                                   unsigned int ncols, unsigned int zero_to,
                                                                   const unsigned int* __restrict__ targets,
@@ -315,7 +317,7 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
 #pragma unroll
   for (int k = 0; k < MAXV; ++k) {
     const unsigned int c = (threadIdx.x + k * CE_FUSED_THREADS) * VEC;
-    q[k] = *reinterpret_cast<const uint4*>(r + (c < whole ? c : last));
+    q[k] = dev_stream_load<STREAM>(reinterpret_cast<const uint4*>(r + (c < whole ? c : last)));
   }
   auto unpack = [](const uint4& w, float (&v)[VEC]) {
     const unsigned int u[4] = {w.x, w.y, w.z, w.w};
@@ -448,7 +450,7 @@ __global__ __launch_bounds__(CE_FUSED_THREADS, 8) void ce_row_fused_kernel(T* __
         w.y = dev_pack_bf16_pair(out[2], out[3]);
         w.z = dev_pack_bf16_pair(out[4], out[5]);
         w.w = dev_pack_bf16_pair(out[6], out[7]);
-        *reinterpret_cast<uint4*>(r + c) = w;
+        dev_stream_store<STREAM>(reinterpret_cast<uint4*>(r + c), w);
       } else {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) out[j] = (c + j == target) ? target_grad : ce_exp<T>(v[j] - m) * scale;
@@ -700,9 +702,10 @@ int32_t omx_linear_cross_entropy_mean(omx_ctx* ctx, const void* x, const void* w
         // One read of the logits tile and one write of the gradient over it.
         OmxKernelTimer timer(ctx, OMX_K_CE, 2.0 * static_cast<double>(nr) * static_cast<double>(nc) * esz);
         // As many 16-byte packs per thread as the row needs (fewer registers for shorter rows).
+        const bool stream = nr * ldt * esz >= CE_STREAM;
         const uint64_t packs = (nc * esz / 16 + CE_FUSED_THREADS - 1) / CE_FUSED_THREADS;
 #define CE_FUSED(T_, P_)                                                                                          \
-  omx_launch_timed(ctx, ce_row_fused_kernel<T_, P_>, grid, block, 0, timer.start(), timer.stop(),                 \
+  omx_launch_timed(ctx, stream ? &ce_row_fused_kernel<T_, P_, true> : &ce_row_fused_kernel<T_, P_, false>, grid, block, 0, timer.start(), timer.stop(),                 \
                    static_cast<T_*>(tile), ldt, r0, static_cast<unsigned>(nc), static_cast<unsigned>(ldt), tg, has_ignore, ignore_index, s.st, \
                    s.valid, ctx->fault, tag)
 #define CE_FUSED_P(T_)                              \

@@ -102,7 +102,11 @@ struct MuonMatrix {
   __device__ __forceinline__ uint64_t iterate(int steps) const { return steps & 1 ? L.xn : L.x; }
 };
 
+template <bool STREAM>
+__device__ __forceinline__ float mu_load(const float* p) { return STREAM ? __builtin_nontemporal_load(p) : *p; }
+
 // buf, the (possibly bf16-rounded) update u, and per-block f64 sums of u^2.
+template <bool STREAM>
 __global__ __launch_bounds__(MU_THREADS) void muon_momentum_kernel(MuonTensors t, MuonWork work, MuonScalars s, OmxFaultWord* fault,
                                                                    unsigned long long tag) {
   __shared__ double red[MU_THREADS];
@@ -118,8 +122,7 @@ __global__ __launch_bounds__(MU_THREADS) void muon_momentum_kernel(MuonTensors t
   double acc = 0.0;
   bool bad = false;
   for (size_t i = begin + threadIdx.x; i < end; i += MU_THREADS) {
-    float gi = g[i];
-    float b = s.mom * m[i] + gi;
+    const float gi = mu_load<STREAM>(g + i), b = s.mom * mu_load<STREAM>(m + i) + gi;
     bad |= !(dev_finite(b) && dev_finite(gi));
     float upd = s.nesterov ? fmaf(s.mom, b, gi) : b;
     if (s.bf16) upd = dev_round_bf16(upd);
@@ -265,6 +268,10 @@ __global__ void muon_apply_kernel(MuonTensors t, MuonWork work, MuonScalars s) {
   }
 }
 
+// Bytes of parameters, gradients, momenta and scratch from which gradients and momenta are read past the caches (48 matrices of 768 x
+// 768: 98 -> 79 us; the update and the momentum just written stay there for the next passes).
+constexpr uint64_t MU_STREAM = 256ull << 20;
+
 // Matrices of one shape that lie one after another in a launch's tables.
 struct MuonRun {
   unsigned first, count;
@@ -347,16 +354,18 @@ int32_t iterate_together(omx_ctx* ctx, const MuonTensors& t, const MuonWork& w, 
 template <typename TX>
 int32_t run_muon(omx_ctx* ctx, const MuonTensors& t, const std::vector<MuonRun>& runs, MuonScalars s, char* ws, bool each, unsigned long long tag) {
   unsigned count = 0;
-  uint64_t most = 0;
+  uint64_t most = 0, total = 0;
   for (const MuonRun& run : runs) {
     count += run.count;
+    total += run.count * run.rows * run.cols;
     most = std::max(most, run.rows * run.cols);
   }
   const MuonWork w{ws, each};
   omx_launch(ctx, muon_clear_flags_kernel, dim3(1, each ? count : 1), dim3(64), 0, t, w);
   OMX_LAUNCH_CHECK(ctx, "muon_clear_flags_kernel");
   const dim3 block(MU_THREADS), over_len(mu_grid(most), count);
-  omx_launch(ctx, muon_momentum_kernel, dim3(static_cast<unsigned>((most + MU_BLOCK - 1) / MU_BLOCK), count), block, 0, t, w, s, ctx->fault, tag);
+  const bool stream = total * 16 >= MU_STREAM;
+  omx_launch(ctx, stream ? &muon_momentum_kernel<true> : &muon_momentum_kernel<false>, dim3(static_cast<unsigned>((most + MU_BLOCK - 1) / MU_BLOCK), count), block, 0, t, w, s, ctx->fault, tag);
   omx_launch(ctx, muon_norm_kernel, dim3(1, count), dim3(1024), 0, t, w, s.bf16, ctx->fault, tag);
   omx_launch(ctx, (muon_normalize_kernel<TX>), over_len, block, 0, t, w);
   OMX_LAUNCH_CHECK(ctx, "muon prologue");

@@ -356,6 +356,49 @@ __device__ __forceinline__ void dev_store<unsigned short>(unsigned short* p, siz
   p[i] = dev_f32_to_bf16_bits(v);
 }
 
+// 16 or 8 bytes that nothing reads again before the caches have forgotten them (STREAM), or as any other load or store. Reading 400 MB
+// out of a set that the 256 MiB memory-side cache does not hold: 6.0 TB/s, 6.6 to 6.9 with the hint.
+template <bool STREAM>
+__device__ __forceinline__ float4 dev_stream_load(const float4* p) {
+  if constexpr (!STREAM) return *p;
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const f4 v = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+template <bool STREAM>
+__device__ __forceinline__ uint2 dev_stream_load(const uint2* p) {
+  if constexpr (!STREAM) return *p;
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 v = __builtin_nontemporal_load(reinterpret_cast<const u2*>(p));
+  return make_uint2(v[0], v[1]);
+}
+template <bool STREAM>
+__device__ __forceinline__ uint4 dev_stream_load(const uint4* p) {
+  if constexpr (!STREAM) return *p;
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  const u4 v = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p));
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+template <bool STREAM>
+__device__ __forceinline__ void dev_stream_store(float4* p, const float4& x) {
+  if constexpr (STREAM) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(f4{x.x, x.y, x.z, x.w}, reinterpret_cast<f4*>(p));
+  } else {
+    *p = x;
+  }
+}
+
+template <bool STREAM>
+__device__ __forceinline__ void dev_stream_store(uint4* p, const uint4& x) {
+  if constexpr (STREAM) {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(u4{x.x, x.y, x.z, x.w}, reinterpret_cast<u4*>(p));
+  } else {
+    *p = x;
+  }
+}
+
 // Four consecutive elements starting at element index i (a multiple of 4; the
 // address must be 16-byte aligned for f32 and 8-byte aligned for bf16).
 template <typename T>

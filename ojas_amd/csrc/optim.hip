@@ -18,6 +18,9 @@
 namespace {
 
 constexpr int OPT_THREADS = 256;
+// Bytes of parameters, gradients and moments from which AdamW reads and writes them past the caches, which a step between two
+// updates has long filled with other things: 124.4 M parameters 682 -> 585 us (6.4 TB/s), 35.5 M 174 -> 156.
+constexpr uint64_t OPT_STREAM = 256ull << 20;
 
 struct AdamWords {
   float decay, one_minus_b1, lerp_high, beta2, one_minus_b2, step_size, bc2_sqrt, eps;
@@ -107,6 +110,7 @@ __global__ __launch_bounds__(OPT_THREADS) void adamw_apply_kernel(float* __restr
 
 // The same update on four consecutive elements per thread (16-byte accesses); every pointer
 // 16-byte aligned (the bf16 copy 8-byte). The last n % 4 elements are thread 0's.
+template <bool STREAM>
 __global__ __launch_bounds__(OPT_THREADS) void adamw_apply_vec_kernel(float* __restrict__ p,
                                                                       const float* __restrict__ g,
                                                                       float* __restrict__ m, float* __restrict__ v,
@@ -123,7 +127,8 @@ __global__ __launch_bounds__(OPT_THREADS) void adamw_apply_vec_kernel(float* __r
   float4* m4 = reinterpret_cast<float4*>(m);
   float4* v4 = reinterpret_cast<float4*>(v);
   for (size_t i = static_cast<size_t>(blockIdx.x) * OPT_THREADS + threadIdx.x; i < quads; i += stride) {
-    const float4 pq = p4[i], gq = g4[i], mq = m4[i], vq = v4[i];
+    const float4 pq = dev_stream_load<STREAM>(p4 + i), gq = dev_stream_load<STREAM>(g4 + i);
+    const float4 mq = dev_stream_load<STREAM>(m4 + i), vq = dev_stream_load<STREAM>(v4 + i);
     const float pi[4] = {pq.x, pq.y, pq.z, pq.w}, gi[4] = {gq.x, gq.y, gq.z, gq.w};
     const float mi[4] = {mq.x, mq.y, mq.z, mq.w}, vi[4] = {vq.x, vq.y, vq.z, vq.w};
     float np[4], nm[4], nv[4];
@@ -133,9 +138,9 @@ __global__ __launch_bounds__(OPT_THREADS) void adamw_apply_vec_kernel(float* __r
       adam_elem(a, pi[e], gi[e], mi[e], vi[e], &np[e], &nm[e], &nv[e], &ok);
       big |= !within_bound(np[e], nm[e], nv[e]);
     }
-    p4[i] = make_float4(np[0], np[1], np[2], np[3]);
-    m4[i] = make_float4(nm[0], nm[1], nm[2], nm[3]);
-    v4[i] = make_float4(nv[0], nv[1], nv[2], nv[3]);
+    dev_stream_store<STREAM>(p4 + i, make_float4(np[0], np[1], np[2], np[3]));
+    dev_stream_store<STREAM>(m4 + i, make_float4(nm[0], nm[1], nm[2], nm[3]));
+    dev_stream_store<STREAM>(v4 + i, make_float4(nv[0], nv[1], nv[2], nv[3]));
     if (p_bf16) {
       uint2 q;
       q.x = dev_pack_bf16_pair(np[0], np[1]);
@@ -482,7 +487,7 @@ static int32_t adamw_impl(omx_ctx* ctx, const char* op, void* param, const void*
                          (reinterpret_cast<uintptr_t>(param_bf16) << 1);
   if ((bits & 15) == 0 && n >= 4) {
     dim3 vec_grid(static_cast<unsigned>((n / 4 + OPT_THREADS - 1) / OPT_THREADS));
-    omx_launch_timed(ctx, adamw_apply_vec_kernel, vec_grid, block, 0, skip_check ? timer.start() : nullptr,
+    omx_launch_timed(ctx, n * 16 >= OPT_STREAM ? &adamw_apply_vec_kernel<true> : &adamw_apply_vec_kernel<false>, vec_grid, block, 0, skip_check ? timer.start() : nullptr,
                      timer.stop(), static_cast<float*>(param), static_cast<const float*>(grad),
                      static_cast<float*>(moment1), static_cast<float*>(moment2), n, a, refuse, unbounded,
                      static_cast<unsigned short*>(param_bf16));
