@@ -87,6 +87,9 @@ void omx_budget_reset_peak(omx_ctx* ctx);
 
 int32_t omx_upload(omx_ctx* ctx, void* dst, uint64_t dst_offset, const void* host_src,
                    uint64_t bytes);
+/* The same without waiting for the copy: `host_src` may be reused on return, `dst` is ordered for work on the context's stream only. */
+int32_t omx_upload_staged(omx_ctx* ctx, void* dst, uint64_t dst_offset, const void* host_src,
+                          uint64_t bytes);
 /* Waits for submitted work, reports a deferred fault, then copies. */
 int32_t omx_download(omx_ctx* ctx, void* host_dst, const void* src, uint64_t src_offset,
                      uint64_t bytes);

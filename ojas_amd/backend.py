@@ -154,9 +154,10 @@ class MiBackend(_native.Methods):
         _native.omx_fill_zero(self._context, t, t.nbytes)
         return t
 
-    def upload(self, host: np.ndarray, dtype: Optional[int] = None) -> DeviceTensor:
+    def upload(self, host: np.ndarray, dtype: Optional[int] = None, staged: bool = False) -> DeviceTensor:
         """BackendCore::upload (backend.rs:917-936). float32 -> F32, uint32 -> U32,
-        uint16 -> BF16 bits; `dtype=BF16` on a float32 array rounds on the device."""
+        uint16 -> BF16 bits; `dtype=BF16` on a float32 array rounds on the device. `staged`: does not wait for the
+        copy, for a tensor that only this backend's ops read (`omx_upload_staged`)."""
         host = np.ascontiguousarray(host)
         if host.dtype == np.float32:
             src_dtype = F32
@@ -170,7 +171,8 @@ class MiBackend(_native.Methods):
             raise OjasError(DTYPE, f"upload of {host.dtype}")
         t = self.empty(host.shape, src_dtype)
         if host.size:
-            _native.omx_upload(self._context, t, 0, host.ctypes.data, host.nbytes)
+            copy = _native.omx_upload_staged if staged else _native.omx_upload
+            copy(self._context, t, 0, host.ctypes.data, host.nbytes)
         if dtype is not None and dtype != src_dtype:
             if src_dtype == F32 and dtype == BF16:
                 return self.to_bf16(t)

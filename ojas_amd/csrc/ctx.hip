@@ -70,6 +70,40 @@ int32_t omx_hip_fail(omx_ctx* ctx, hipError_t err, const char* what) {
   return omx_fail(ctx, st, "hip: %s failed: %s (%d)", what, hipGetErrorString(err), code);
 }
 
+namespace {
+constexpr uint64_t kReadback = 4096, kStage = 1ull << 20, kStageMost = 256ull << 10;
+char* readback(omx_ctx* ctx) { return reinterpret_cast<char*>(ctx->fault_host) + 64; }
+
+// The fault word and `n` bytes of `src` into pinned host memory.
+__global__ __launch_bounds__(256) void read_back_kernel(const OmxFaultWord* fault, OmxFaultWord* fault_host, const char* src, char* dst, int n) {
+  if (threadIdx.x == 0) *fault_host = *fault;
+  for (int i = threadIdx.x; i < n; i += 256) dst[i] = src[i];
+}
+// Out of pinned host memory, 16 bytes a thread (both 16-byte aligned) and what is left of them.
+__global__ __launch_bounds__(256) void stage_kernel(const char* src, char* dst, int n) {
+  const int at = (blockIdx.x * 256 + threadIdx.x) * 16;
+  if (at + 16 <= n) *reinterpret_cast<uint4*>(dst + at) = *reinterpret_cast<const uint4*>(src + at);
+  else
+    for (int i = at; i < n; ++i) dst[i] = src[i];
+}
+
+// Whether these bytes lie in one of the context's own blocks. What else a caller names (a range past its block, another device's
+// memory, a host pointer) keeps the runtime's copy and its checks.
+bool own_range(const omx_ctx* ctx, const void* at, uint64_t n) {
+  auto block = ctx->allocations.upper_bound(const_cast<void*>(at));
+  if (block == ctx->allocations.begin()) return false;
+  --block;
+  const uint64_t from = static_cast<uint64_t>(static_cast<const char*>(at) - static_cast<const char*>(block->first));
+  return from <= block->second && n <= block->second - from;
+}
+
+int32_t wait(omx_ctx* ctx) {
+  OMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->staged = 0;
+  return OMX_OK;
+}
+}  // namespace
+
 static int32_t reset_fault(omx_ctx* ctx) {
   ctx->fault_host->mask = 0;
   ctx->fault_host->first = ~0ull;
@@ -107,7 +141,7 @@ int32_t omx_open(int32_t device, uint64_t budget_bytes, omx_ctx** out) {
     return OMX_UNSUPPORTED;
   }
   if (hipStreamCreate(&ctx->stream) != hipSuccess || hipMalloc(&ctx->fault, 256) != hipSuccess ||
-      hipHostMalloc(&ctx->fault_host, sizeof(OmxFaultWord)) != hipSuccess) {
+      hipHostMalloc(&ctx->fault_host, 64 + kReadback) != hipSuccess) {
     delete ctx;
     return OMX_BACKEND;
   }
@@ -134,6 +168,7 @@ void omx_close(omx_ctx* ctx) {
   for (auto& kv : ctx->pool) (void)hipFree(kv.second);
   if (ctx->fault) (void)hipFree(ctx->fault);
   if (ctx->fault_host) (void)hipHostFree(ctx->fault_host);
+  if (ctx->stage) (void)hipHostFree(ctx->stage);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -280,11 +315,41 @@ int32_t omx_upload(omx_ctx* ctx, void* dst, uint64_t dst_offset, const void* hos
   return OMX_OK;
 }
 
-int32_t omx_sync(omx_ctx* ctx) {
+// For inputs that only work on this stream reads (a step's tokens): no wait. An upload and its wait were some 12 us in which a small
+// model's step had not begun.
+int32_t omx_upload_staged(omx_ctx* ctx, void* dst, uint64_t dst_offset, const void* host_src, uint64_t bytes) {
   OMX_REQUIRE_CTX(ctx);
-  OMX_HIP(ctx, hipMemcpyAsync(ctx->fault_host, ctx->fault, sizeof(OmxFaultWord), hipMemcpyDeviceToHost,
-                              ctx->stream));
-  OMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  char* to = static_cast<char*>(dst) + dst_offset;
+  if (!dst || !host_src || bytes == 0 || bytes > kStageMost || (reinterpret_cast<uintptr_t>(to) & 15u) || capturing(ctx) ||
+      !own_range(ctx, to, bytes))
+    return omx_upload(ctx, dst, dst_offset, host_src, bytes);
+  if (!ctx->stage && hipHostMalloc(&ctx->stage, kStage) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->stage = nullptr;
+    return omx_upload(ctx, dst, dst_offset, host_src, bytes);
+  }
+  if (ctx->staged + bytes > kStage) {
+    const int32_t rc = wait(ctx);
+    if (rc != OMX_OK) return rc;
+  }
+  char* from = ctx->stage + ctx->staged;
+  memcpy(from, host_src, bytes);
+  omx_launch(ctx, stage_kernel, dim3(static_cast<unsigned>((bytes + 4095) / 4096)), dim3(256), 0, from, to, static_cast<int>(bytes));
+  OMX_LAUNCH_CHECK(ctx, "stage_kernel");
+  ctx->staged += (bytes + 255) & ~255ull;
+  return OMX_OK;
+}
+
+}  // extern "C"
+
+namespace {
+// Waits for submitted work and reports a deferred fault; with the fault word come `n` (at most kReadback) bytes of `src`, to readback().
+// One launch and one wait: a copy of the fault word, a wait, a copy of the value and a wait were some 25 us between two halves of a step.
+int32_t sync_with(omx_ctx* ctx, const void* src, uint64_t n) {
+  omx_launch(ctx, read_back_kernel, dim3(1), dim3(256), 0, ctx->fault, ctx->fault_host, static_cast<const char*>(src), readback(ctx), static_cast<int>(n));
+  OMX_LAUNCH_CHECK(ctx, "read_back_kernel");
+  const int32_t waited = wait(ctx);
+  if (waited != OMX_OK) return waited;
   if (ctx->fault_host->mask != 0) {
     uint32_t op = static_cast<uint32_t>(ctx->fault_host->first & 0x7full);
     bool range = (ctx->fault_host->first & 0x80ull) != 0;
@@ -295,15 +360,27 @@ int32_t omx_sync(omx_ctx* ctx) {
   }
   return OMX_OK;
 }
+}  // namespace
+
+extern "C" {
+
+int32_t omx_sync(omx_ctx* ctx) {
+  OMX_REQUIRE_CTX(ctx);
+  return sync_with(ctx, nullptr, 0);
+}
 
 int32_t omx_download(omx_ctx* ctx, void* host_dst, const void* src, uint64_t src_offset, uint64_t bytes) {
   OMX_REQUIRE_CTX(ctx);
   if (!host_dst || !src) return omx_fail(ctx, OMX_PLACEMENT, "download: null pointer");
-  int32_t rc = omx_sync(ctx);
-  if (rc != OMX_OK) return rc;
-  if (bytes == 0) return OMX_OK;
-  OMX_HIP(ctx, hipMemcpyAsync(host_dst, static_cast<const char*>(src) + src_offset, bytes, hipMemcpyDeviceToHost,
-                              ctx->stream));
+  const char* from = static_cast<const char*>(src) + src_offset;
+  const bool small = bytes <= kReadback && own_range(ctx, from, bytes);
+  const int32_t rc = sync_with(ctx, from, small ? bytes : 0);
+  if (rc != OMX_OK || bytes == 0) return rc;
+  if (small) {
+    memcpy(host_dst, readback(ctx), bytes);
+    return OMX_OK;
+  }
+  OMX_HIP(ctx, hipMemcpyAsync(host_dst, from, bytes, hipMemcpyDeviceToHost, ctx->stream));
   OMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return OMX_OK;
 }

@@ -84,7 +84,10 @@ struct omx_ctx {
   std::multimap<uint64_t, void*> pool;
   uint64_t pooled_bytes = 0;
   OmxFaultWord* fault = nullptr;  // device
-  OmxFaultWord* fault_host = nullptr;  // pinned
+  OmxFaultWord* fault_host = nullptr;  // pinned, with kReadback bytes for what a small download brings behind it
+  // Pinned memory that small uploads pass through (omx_upload_staged), taken by the first; up to `staged` the stream may still read it.
+  char* stage = nullptr;
+  uint64_t staged = 0;
   unsigned int* kv_refused = nullptr;  // device, behind the fault word: KvWrite::refused, zero between calls
   uint64_t sequence = 0;
   std::string last_error;

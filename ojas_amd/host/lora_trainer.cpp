@@ -495,8 +495,8 @@ int32_t olora_init_adapters(olora* t, uint64_t seed, float std) {
 
 int32_t olora_set_batch(olora* t, const uint32_t* ids, const uint32_t* targets) {
   if (!t || !ids || !targets) return OMX_BACKEND;
-  TRY(omx_upload(t->ctx, t->ids, 0, ids, t->N * 4));
-  TRY(omx_upload(t->ctx, t->targets, 0, targets, t->N * 4));
+  TRY(omx_upload_staged(t->ctx, t->ids, 0, ids, t->N * 4));
+  TRY(omx_upload_staged(t->ctx, t->targets, 0, targets, t->N * 4));
   return OMX_OK;
 }
 

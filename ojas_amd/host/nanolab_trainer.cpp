@@ -857,8 +857,8 @@ int32_t onano_init_reference(onano* t, uint64_t seed) {
 int32_t onano_micro_batch(onano* t, const uint32_t* ids, const uint32_t* targets, float loss_seed, float loss_scale,
                           int32_t first) {
   if (!t || !ids || !targets) return OMX_BACKEND;
-  TRY(omx_upload(t->ctx, t->ids, 0, ids, t->N * 4));
-  TRY(omx_upload(t->ctx, t->targets, 0, targets, t->N * 4));
+  TRY(omx_upload_staged(t->ctx, t->ids, 0, ids, t->N * 4));
+  TRY(omx_upload_staged(t->ctx, t->targets, 0, targets, t->N * 4));
   return micro_batch(t, loss_seed, loss_scale, first);
 }
 

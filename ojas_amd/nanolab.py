@@ -290,13 +290,16 @@ class NanolabTrainer:
         uniform = all(c == live[0] for c in live)
         total = sum(counts)
         acc, loss_sum = None, None
+        # (A subclass or wrapper of the backend, which may count, tag or check calls, gets the calls it knows.)
+        together = type(be.inner if self.autocast else be) is MiBackend
+        staged = {"staged": True} if together else {}
         for (ids, targets), count in zip(batches, counts):
             if count == 0:
                 continue
             weight = float(np.float32(1.0 / len(live))) if uniform else float(np.float32(count / total))
             with (be.region() if self.autocast else nullcontext()):
-                loss, _, grads = self.graph.loss_and_grads(be.upload(np.ascontiguousarray(ids, np.uint32)),
-                                                           be.upload(np.ascontiguousarray(targets, np.uint32)),
+                loss, _, grads = self.graph.loss_and_grads(be.upload(np.ascontiguousarray(ids, np.uint32), **staged),
+                                                           be.upload(np.ascontiguousarray(targets, np.uint32), **staged),
                                                            loss_seed=weight)
             if acc is None:
                 acc = {n: grads[n] for n in self.trainable}
@@ -309,8 +312,6 @@ class NanolabTrainer:
         # One set of launches for the matrices of all shapes, one for everything AdamW steps: a tensor at a time, a small
         # model's 32 matrices took 990 launches and its 25 vectors 75, most of the step's time.
         cfg = MuonNs5Config(self.matrix_lr * lr_multiplier, MUON_MOMENTUM, MUON_WEIGHT_DECAY, 1, int(self.ns5_bf16))
-        # (A subclass or wrapper of the backend, which may count, tag or check calls, gets one for each shape.)
-        together = type(be.inner if self.autocast else be) is MiBackend
         for names in [sum(self.muon_groups, [])] if together and self.muon_groups else self.muon_groups:
             step = be.muon_ns5_step_shapes if together else be.muon_ns5_step_list
             step([self.params[n] for n in names], [acc[n] for n in names], [self.state[n][0] for n in names], cfg)
