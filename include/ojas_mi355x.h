@@ -118,6 +118,10 @@ int32_t omx_linear_backward(omx_ctx* ctx, const void* x, const void* w, const vo
                             int32_t operand_dtype, void* gx, int32_t gx_dtype, void* gw,
                             int32_t gw_dtype, uint64_t rows, uint64_t in_features,
                             uint64_t out_features);
+/* The same with gx (f32, required) added to: where several projections read one input. */
+int32_t omx_linear_backward_onto(omx_ctx* ctx, const void* x, const void* w, const void* gy,
+                                 int32_t operand_dtype, void* gx, void* gw, int32_t gw_dtype, uint64_t rows,
+                                 uint64_t in_features, uint64_t out_features);
 /* General product behind the three above and the Newton-Schulz products:
  * C[m,n] (+)= A.B with A(i,p) at a[i*a_rs + p*a_cs], B(p,j) at b[p*b_rs + j*b_cs]
  * (element strides; one stride of each operand must be 1). */
@@ -688,6 +692,8 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * between one 128-row block per workgroup and a mirrored pair by how the pairs fill the chip
  * (default) and split a block's tiles over groups of waves where workgroups are few, 1 / 2 = always one block / always the
  * pair, 3 / 4 = always two / four groups (two at head_dim 128; the parity tests run all).
+ * "gemm_f32_pair": -1 = both f32 gradients of omx_linear_backward go out in one launch where that is estimated to take less
+ * (default), 0 = never, 1 .. 4 = always on one of four pairs of tiles, where the operands' alignment allows;
  * "gemm_f32": -1 = f32 products take the tile with the least estimated time (default), 0 .. 4 = always the register-fragment
  * kernel's 16 x 16 / 16 x 32 / 32 x 32 / 64 x 32 / 64 x 64 tile, 5 .. 8 = the direct-to-LDS kernel's 64 x 64 / 64 x 32 / 64 x 32 by
  * two wave groups / 32 x 32 by four, wherever the operands fit it, 9 = the register-staged kernel.

@@ -83,6 +83,7 @@ extern "C" {
     pub fn omx_to_f32(ctx: *mut OmxCtx, x_bf16: *const c_void, y_f32: *mut c_void, n: u64) -> i32;
     pub fn omx_linear_forward(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, w: *const c_void, w_dtype: i32, y: *mut c_void, y_dtype: i32, rows: u64, in_features: u64, out_features: u64) -> i32;
     pub fn omx_linear_backward(ctx: *mut OmxCtx, x: *const c_void, w: *const c_void, gy: *const c_void, operand_dtype: i32, gx: *mut c_void, gx_dtype: i32, gw: *mut c_void, gw_dtype: i32, rows: u64, in_features: u64, out_features: u64) -> i32;
+    pub fn omx_linear_backward_onto(ctx: *mut OmxCtx, x: *const c_void, w: *const c_void, gy: *const c_void, operand_dtype: i32, gx: *mut c_void, gw: *mut c_void, gw_dtype: i32, rows: u64, in_features: u64, out_features: u64) -> i32;
     pub fn omx_gemm(ctx: *mut OmxCtx, a: *const c_void, a_rs: u64, a_cs: u64, b: *const c_void, b_rs: u64, b_cs: u64, operand_dtype: i32, c: *mut c_void, c_dtype: i32, m: u64, k: u64, n: u64, accumulate: i32) -> i32;
     pub fn omx_gemm_pitched(ctx: *mut OmxCtx, a: *const c_void, a_rs: u64, a_cs: u64, b: *const c_void, b_rs: u64, b_cs: u64, operand_dtype: i32, c: *mut c_void, c_dtype: i32, ldc: u64, m: u64, k: u64, n: u64, accumulate: i32) -> i32;
     pub fn omx_gemm_strided_batch(ctx: *mut OmxCtx, a: *const c_void, a_rs: u64, a_cs: u64, b: *const c_void, b_rs: u64, b_cs: u64, operand_dtype: i32, c: *mut c_void, c_dtype: i32, m: u64, k: u64, n: u64, accumulate: i32, count: u64, stride_a: u64, stride_b: u64, stride_c: u64) -> i32;

@@ -240,6 +240,15 @@ class MiBackend(_native.Methods):
         _native.omx_linear_backward(self._context, x, w, gy, x.dtype, gx, gx_dtype, gw, F32, rows, kin, nout)
         return gx, gw
 
+    def linear_backward_onto(self, g, x, w, gy):
+        """g (f32, written to) + the input gradient of `linear_backward`, and its weight gradient."""
+        rows, kin, nout = x.numel // x.shape[-1], x.shape[-1], w.shape[0]
+        if g.shape != x.shape or g.dtype != F32 or not (x.dtype == w.dtype == gy.dtype):
+            raise OjasError(DTYPE, "linear_backward_onto: an f32 sum of the input's shape, operands that share a dtype")
+        gw = self.empty(w.shape, F32)
+        _native.omx_linear_backward_onto(self._context, x, w, gy, x.dtype, g, gw, F32, rows, kin, nout)
+        return g, gw
+
     def linear_backward_input(self, w, gy, in_features=None, gx_dtype=F32):
         rows = gy.numel // gy.shape[-1]
         kin, nout = w.shape[1], w.shape[0]

@@ -338,6 +338,10 @@ int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);
 // f32 kernels: small outputs (gemm_frag32.hip) and direct-to-LDS loads (gemm_dma32.hip; g.K counts whole 32-column steps).
 // `_us`: what a tile is estimated to take; negative: not one for it.
 constexpr int FRAG32_TILES = 5, DMA32_TILES = 4;
+// x: A k-contiguous, B k-major; w: both k-major. Estimate of a call of both (< 0: the tile does not fit), launch.
+constexpr int FRAG32_PAIRS = 4;
+double omx_gemm_frag32_pair_us(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w, int tile);
+int32_t omx_gemm_frag32_pair(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w, int tile);
 double omx_gemm_frag32_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
 int32_t omx_gemm_frag32_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
 // Independent f32 products C = A.B, or s1 aux + s2 A.B where `aux` is set (C's layout), in one launch; strides in elements, as

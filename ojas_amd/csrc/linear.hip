@@ -71,6 +71,12 @@ int32_t omx_linear_backward(omx_ctx* ctx, const void* x, const void* w, const vo
   if (gx && !w) return omx_fail(ctx, OMX_PLACEMENT, "%s: weight is null", op);
   if (gw && !x) return omx_fail(ctx, OMX_PLACEMENT, "%s: input is null", op);
   if (rows == 0 || in_features == 0 || out_features == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
+  if (gx && gw && operand_dtype == OMX_F32 && gx_dtype == OMX_F32 && gw_dtype == OMX_F32) {
+    int32_t rc = OMX_OK;
+    if (omx_linear_backward_pair(ctx, static_cast<const float*>(x), static_cast<const float*>(w), static_cast<const float*>(gy),
+                                 static_cast<float*>(gx), static_cast<float*>(gw), rows, in_features, out_features, false, &rc))
+      return rc;
+  }
   if (gx) {
     // gx(i,j) = sum_o gy[i*out + o] * W[o*in + j]
     int32_t rc = omx_gemm_impl(ctx, F_LINEAR_BACKWARD, gy, out_features, 1, w, in_features, 1, operand_dtype, gx,
@@ -84,6 +90,22 @@ int32_t omx_linear_backward(omx_ctx* ctx, const void* x, const void* w, const vo
     if (rc != OMX_OK) return rc;
   }
   return OMX_OK;
+}
+
+// The tape's fan-in at a projection's input (ojas-autograd/src/tape.rs:2565-2591): gx += gy.W behind gw = gy^T.x.
+int32_t omx_linear_backward_onto(omx_ctx* ctx, const void* x, const void* w, const void* gy, int32_t operand_dtype, void* gx, void* gw,
+                                 int32_t gw_dtype, uint64_t rows, uint64_t in_features, uint64_t out_features) {
+  OMX_REQUIRE_CTX(ctx);
+  if (gx && gw && x && w && gy && rows && in_features && out_features && operand_dtype == OMX_F32 && gw_dtype == OMX_F32) {
+    int32_t rc = OMX_OK;
+    if (omx_linear_backward_pair(ctx, static_cast<const float*>(x), static_cast<const float*>(w), static_cast<const float*>(gy),
+                                 static_cast<float*>(gx), static_cast<float*>(gw), rows, in_features, out_features, true, &rc))
+      return rc;
+  }
+  const int32_t rc = omx_linear_backward(ctx, x, nullptr, gy, operand_dtype, nullptr, operand_dtype, gw, gw_dtype, rows, in_features,
+                                         out_features);
+  if (rc != OMX_OK) return rc;
+  return omx_gemm(ctx, gy, out_features, 1, w, in_features, 1, operand_dtype, gx, OMX_F32, rows, out_features, in_features, 1);
 }
 
 // linear_forward followed by gelu (ojas-model block: up-projection then activation), the

@@ -114,6 +114,7 @@ struct omx_ctx {
   int gemm_dma_mode = 1;
   int q8_widen = -1;         // int8 products over a widened copy of the weight: -1 by rule, 0 never, 1 wherever they can
   int gemm_f32_tile = -1;    // f32 products: -1: choose by estimate; 0..4, 5..8: a tile of gemm_frag32.hip, gemm_dma32.hip; 9: the register-staged kernel
+  int gemm_f32_pair = -1;    // both f32 gradients of a linear layer in one launch: -1: by estimate; 0: never; 1..4: on these tiles
   int gemm_row_split = 1;    // 0: a product whose last round of 256 x 256 tiles is mostly empty is not cut by rows
   bool gemm_in_row_split = false;  // set while omx_gemm_impl runs the two halves of a cut product
   int gemm_forced_tiling = -1;     // the tiling the first half keeps, whatever its own tile count says
@@ -246,6 +247,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
                       uint64_t b_rs, uint64_t b_cs, int32_t operand_dtype, void* c, int32_t c_dtype, uint64_t ldc,
                       uint64_t m, uint64_t k, uint64_t n, int32_t accumulate, const OmxGemmEpilogue* epi = nullptr,
                       const OmxGemmBatch* batch = nullptr, uint64_t a_k = 0, const OmxLowRank* low_rank = nullptr);
+bool omx_linear_backward_pair(omx_ctx* ctx, const float* x, const float* w, const float* gy, float* gx, float* gw, uint64_t rows, uint64_t in,
+                              uint64_t out, bool onto, int32_t* rc);
 double omx_gemm_bf16_us(const omx_ctx* ctx, uint64_t m, uint64_t k, uint64_t n);
 // Whether omx_gemm_impl takes a bf16 product k-contiguous in A with a low-rank term (on the direct-to-LDS kernels).
 bool omx_gemm_takes_low_rank(const omx_ctx* ctx, const void* a, uint64_t lda, const void* b, uint64_t ldb, uint64_t k);

@@ -456,7 +456,7 @@ struct Symbol {
 
 #define OMX_ENTRIES(X)                                                                                                   \
   X(omx_fill_zero) X(omx_upload) X(omx_upload_staged) X(omx_download) X(omx_sync) X(omx_cast_bf16) X(omx_to_bf16) X(omx_to_f32)               \
-  X(omx_linear_forward) X(omx_linear_backward) X(omx_gemm) X(omx_gemm_strided_batch) X(omx_gemm_pitched_strided_batch)   \
+  X(omx_linear_forward) X(omx_linear_backward) X(omx_linear_backward_onto) X(omx_gemm) X(omx_gemm_strided_batch) X(omx_gemm_pitched_strided_batch)   \
   X(omx_linear_i8_group_forward) X(omx_linear_i8_group_backward_input) X(omx_pack_i8_group)                              \
   X(omx_causal_sdpa_forward) X(omx_causal_sdpa_backward) X(omx_causal_sdpa_backward_recompute)                           \
   X(omx_linear_gelu_forward) X(omx_linear_backward_input_gelu) X(omx_causal_attention_forward)                           \

@@ -123,9 +123,7 @@ class NanolabGraph:
         def linear_backward_onto(g, x, w, gy):
             """g (which is no one else's) + the projection's input gradient, and its weight gradient."""
             if fused:
-                _, gw = be.linear_backward(x, w, gy, need_gx=False)
-                nout, kin = w.shape
-                return be.gemm(gy, (nout, 1), w, (kin, 1), N, nout, kin, c=g), gw
+                return be.linear_backward_onto(g, x, w, gy)
             part, gw = be.linear_backward(x, w, gy)
             return be.residual_add_forward(g, part), gw
 

@@ -703,3 +703,45 @@ def test_f32_activation_in_the_store_pass_is_named_as_the_separate_pass_is(be, t
         be.sync()
     finally:
         be.set_option("gemm_f32", -1)
+
+
+@pytest.mark.parametrize("pair", [1, 2, 3, 4, -1])
+@pytest.mark.parametrize("rows,kin,nout", [(1, 4, 4), (16, 32, 16), (65, 34, 20), (130, 96, 36), (257, 70, 12), (1021, 66, 132), (300, 512, 260), (4100, 32, 64)])
+def test_both_gradients_in_one_launch(be, pair, rows, kin, nout):
+    """Each pair of tiles, forced where it fits, and the rule's choice: outputs that end inside a tile, walks of one step, of fewer
+    steps than waves and ending inside one, more tiles than compute units; against the f64 products, k products and k sums rounded
+    to f32 each: (k + 1) 2^-24 sum |a||b|. A value that is not finite is named; outputs that overlap an operand take two launches."""
+    from ojas_amd.backend import OjasError
+
+    print(f"gradients together {pair} {rows}x{kin}x{nout}", flush=True)
+    be.set_option("gemm_dma", 1)
+    r = np.random.default_rng(rows + kin + nout)
+    x, w, gy = (r.normal(size=s).astype(np.float32) for s in ((rows, kin), (nout, kin), (rows, nout)))
+    x64, w64, g64 = (a.astype(np.float64) for a in (x, w, gy))
+    bounds = [(nout + 1) * 2.0 ** -24 * (np.abs(g64) @ np.abs(w64)), (rows + 1) * 2.0 ** -24 * (np.abs(g64).T @ np.abs(x64))]
+    dx, dw, dg = (be.upload(a) for a in (x, w, gy))
+    be.set_option("gemm_f32_pair", pair)
+    try:
+        for got, want, bound in zip(be.linear_backward(dx, dw, dg), (g64 @ w64, g64.T @ x64), bounds):
+            assert (np.abs(be.download(got) - want) <= bound + 1e-30).all()
+        before = r.normal(size=x.shape).astype(np.float32)
+        onto, gw = be.linear_backward_onto(be.upload(before), dx, dw, dg)
+        assert (np.abs(be.download(onto) - (g64 @ w64 + before)) <= bounds[0] * (nout + 2) / (nout + 1) + 2.0 ** -23 * np.abs(before)).all()
+        assert (np.abs(be.download(gw) - g64.T @ x64) <= bounds[1] + 1e-30).all()
+        n64 = tuple(C.c_uint64(v) for v in (rows, kin, nout))
+        back = lambda gx: be._check(be._lib.omx_linear_backward(be._ctx, be._p(dx), be._p(dw), be._p(dg), C.c_int32(0), be._p(gx), C.c_int32(0),
+                                                                be._p(gw), C.c_int32(0), *n64))
+        be.set_option("gemm_f32_pair", 0)
+        back(dx)  # over the layer's input, which the second product then reads
+        apart = be.download(gw)
+        dx = be.upload(x)
+        be.set_option("gemm_f32_pair", pair)
+        back(dx)
+        assert np.array_equal(be.download(gw), apart)
+        gy[-1, -1] = np.inf
+        be.linear_backward(be.upload(x), dw, be.upload(gy))
+        with pytest.raises(OjasError) as e:
+            be.sync()
+        assert e.value.detail == "linear_backward"
+    finally:
+        be.set_option("gemm_f32_pair", -1)
