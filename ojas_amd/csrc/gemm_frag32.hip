@@ -13,7 +13,7 @@
 // 4 g + j of the lanes' groups g = lane / 16, from both operands alike. A k-contiguous operand's lane then
 // loads 16 bytes of its row. A k-major one loads, for each j, MB (NB) adjacent rows of K row 4 g + j in one
 // piece: its blocks interleave, block m holding rows MB i + m, so one load serves every block.
-#include "gemm_tiles.h"
+#include "gemm_dma32_impl.h"
 
 namespace {
 
@@ -244,15 +244,19 @@ __global__ __launch_bounds__(PAIR_WAVES * 64) void gemm_frag32_pair_kernel(GemmA
 // 3 to 13 us and leaves most of the chip idle: the k-th products of all chains go out together. 32 x 32 tiles whose four waves share
 // K. Four blocks of d = 256 (32 matrices): 33, 26 and 40 us for the first, second and third products of an iteration, 20, 13 and 28
 // in one launch each; bound by the waits of short walks over K (a third of the f32 matrix rate). 64 x 32 tiles took 22, 16 and 30,
-// steps of 32 K values with all of a step's loads together 28, 16 and 33.
+// steps of 32 K values with all of a step's loads together 28, 16 and 33. The third products, whose outputs are the matrices, go on
+// gemm_dma32.hip's 64 x 64 tiles instead where those make half a workgroup per compute unit (28 -> 23 us: half the operand bytes a
+// product; a step of the 32 matrices 337 -> 308 us, of 64 556 -> 508, 16 matrices 240 -> 237).
 // `symmetric`: the output equals its transpose (X X^T, A A and their sums with a symmetric tensor): tiles below the diagonal are
 // written from those above it, the same sums in the same order.
-constexpr int GROUP_WAVES = 4, GROUP_TILE = 32;
+constexpr int GROUP_WAVES = 4, GROUP_TILE = 32, GROUP_DMA = 4, GROUP_DMA_TILE = 64;
+constexpr int GROUP_LDS = 2 * 2 * GROUP_DMA_TILE * 128;  // two stages of two operands
+static_assert(GROUP_LDS >= GROUP_WAVES * GROUP_TILE * (GROUP_TILE + 4) * 4, "the waves' sums fit");
 struct FragProduct {
   const float *a, *b, *aux;
   float* c;
   long lda, ldb, ldc, batch;  // batch: BYTES between the products of a strided batch, in every operand
-  int M, N, K, tiles_m, tiles_n, batches, layout, c_vec;  // layout: 2 A k-major + B k-major
+  int M, N, K, tiles_m, tiles_n, batches, layout, c_vec;  // layout: 2 A k-major + B k-major; GROUP_DMA: 64 x 64 tiles
 };
 struct FragGroup {
   FragProduct product[FRAG32_GROUP];
@@ -263,7 +267,8 @@ struct FragGroup {
   unsigned long long tag;
 };
 __global__ __launch_bounds__(GROUP_WAVES * 64) void gemm_frag32_group_kernel(FragGroup q) {
-  __shared__ __align__(16) float sums[GROUP_WAVES * GROUP_TILE * (GROUP_TILE + 4)];
+  __shared__ __attribute__((aligned(1024))) char smem[GROUP_LDS];
+  float* const sums = reinterpret_cast<float*>(smem);  // [GROUP_WAVES][GROUP_TILE][GROUP_TILE + 4]
   constexpr int PITCH32 = GROUP_TILE + 4;
   int which = 0;  // (all of `first` in one load)
 #pragma unroll
@@ -271,22 +276,32 @@ __global__ __launch_bounds__(GROUP_WAVES * 64) void gemm_frag32_group_kernel(Fra
   const FragProduct& p = q.product[which];
   const int total = p.tiles_m * p.tiles_n, index = blockIdx.x - q.first[which];
   if (index >= total * p.batches) return;
-  const int r = tile_of_eighth(index, total * p.batches), product = r / total, id = r - product * total;
-  const int tile_m = id / p.tiles_n, tile_n = id - tile_m * p.tiles_n;
-  if (q.symmetric && tile_m > tile_n) return;
   GemmArgs g;
-  const long shift = product * p.batch;
-  g.a = reinterpret_cast<const char*>(p.a) + shift;
-  g.b = reinterpret_cast<const char*>(p.b) + shift;
-  g.c = reinterpret_cast<char*>(p.c) + shift;
-  g.aux_in = p.aux ? reinterpret_cast<const unsigned short*>(reinterpret_cast<const char*>(p.aux) + shift) : nullptr;
+  g.a = p.a;
+  g.b = p.b;
+  g.c = p.c;
+  g.aux_in = reinterpret_cast<const unsigned short*>(p.aux);
+  g.aux_out = nullptr;
   g.lda = p.lda; g.ldb = p.ldb; g.ldc = p.ldc;
-  g.M = p.M; g.N = p.N; g.K = p.K;
+  g.M = p.M; g.N = p.N; g.K = g.k_rows = p.K;
+  g.tiles_m = p.tiles_m; g.tiles_n = p.tiles_n;
+  g.batches = p.batches;
+  g.batch_a = g.batch_b = g.batch_c = p.batch;
   g.c_bf16 = 0;
   g.accumulate = p.aux ? 2 : 0;
   g.c_vec = p.c_vec;
   g.splits = 1;
   g.epi_s1 = q.s1; g.epi_s2 = q.s2;
+  g.fault = q.fault;
+  g.tag = g.act_tag = q.tag;
+  if (p.layout == GROUP_DMA) {  // (uniform)
+    dma32_tile<false, true, 2, 2, 2, 2, 2, 1, false, 0>(g, index, smem);
+    return;
+  }
+  const int r = tile_of_eighth(index, total * p.batches), product = r / total, id = r - product * total;
+  const int tile_m = id / p.tiles_n, tile_n = id - tile_m * p.tiles_n;
+  if (q.symmetric && tile_m > tile_n) return;
+  gemm_select_batch(g, product);
   const int row0 = tile_m * GROUP_TILE, col0 = tile_n * GROUP_TILE;
   switch (p.layout) {  // (uniform)
     case 0: frag32_sums<false, false, 2, 2, GROUP_WAVES, true>(g, row0, col0, sums); break;
@@ -452,6 +467,12 @@ static bool group_fits(const OmxGemmProduct& p) {
          frag_fits(a_km, p.a, lda, static_cast<int>(p.m), 2, 0) && frag_fits(b_km, p.b, ldb, static_cast<int>(p.n), 2, 0);
 }
 
+// A k-contiguous, B k-major, whole steps of 32 and aligned pieces.
+static bool group_fits_dma(const OmxGemmProduct& p) {
+  return p.a_cs == 1 && p.b_cs == 1 && p.b_rs != 1 && p.k % 32 == 0 && p.n % 4 == 0 && p.a_rs % 4 == 0 && p.b_rs % 4 == 0 && p.a_rs <= 1u << 22 &&
+         p.b_rs <= 1u << 22 && ((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b)) & 15u) == 0;
+}
+
 int32_t omx_gemm_frag32_group(omx_ctx* ctx, const OmxGemmProduct* products, int count, bool symmetric, float s1, float s2, unsigned long long tag) {
   FragGroup q;
   q.symmetric = symmetric;
@@ -459,6 +480,11 @@ int32_t omx_gemm_frag32_group(omx_ctx* ctx, const OmxGemmProduct* products, int 
   q.s2 = s2;
   q.fault = ctx->fault;
   q.tag = tag;
+  uint64_t large_tiles = 0;
+  for (int i = 0; i < count && !symmetric; ++i)
+    if (group_fits_dma(products[i]))
+      large_tiles += ((products[i].m + GROUP_DMA_TILE - 1) / GROUP_DMA_TILE) * ((products[i].n + GROUP_DMA_TILE - 1) / GROUP_DMA_TILE) * products[i].batches;
+  const bool large = 2 * large_tiles >= static_cast<uint64_t>(ctx->cu_count > 0 ? ctx->cu_count : 256);
   int at = 0;
   for (int i = 0; i < count; ++i) {
     const OmxGemmProduct& p = products[i];
@@ -471,10 +497,11 @@ int32_t omx_gemm_frag32_group(omx_ctx* ctx, const OmxGemmProduct* products, int 
     f.ldc = static_cast<long>(p.ldc);
     f.batch = static_cast<long>(p.stride) * 4;
     f.M = static_cast<int>(p.m); f.N = static_cast<int>(p.n); f.K = static_cast<int>(p.k);
-    f.tiles_m = (f.M + GROUP_TILE - 1) / GROUP_TILE;
-    f.tiles_n = (f.N + GROUP_TILE - 1) / GROUP_TILE;
     f.batches = static_cast<int>(p.batches);
-    f.layout = 2 * a_km + b_km;
+    f.layout = large && !a_km && b_km && group_fits_dma(p) ? GROUP_DMA : 2 * a_km + b_km;
+    const int tile = f.layout == GROUP_DMA ? GROUP_DMA_TILE : GROUP_TILE;
+    f.tiles_m = (f.M + tile - 1) / tile;
+    f.tiles_n = (f.N + tile - 1) / tile;
     f.c_vec = (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0 && p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.aux) & 15u) == 0;
     q.first[i] = at;
     at += (f.tiles_m * f.tiles_n * f.batches + 7) & ~7;

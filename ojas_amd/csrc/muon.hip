@@ -341,7 +341,7 @@ int32_t iterate_together(omx_ctx* ctx, const MuonTensors& t, const MuonWork& w, 
         if (stage == 0) products[i] = tall ? OmxGemmProduct{x, 1, cols, x, cols, 1, am, r, r, c, r, nullptr, run.count, es}
                                            : OmxGemmProduct{x, cols, 1, x, 1, cols, am, r, r, c, r, nullptr, run.count, es};
         else if (stage == 1) products[i] = OmxGemmProduct{am, r, 1, am, r, 1, a2, r, r, r, r, am, run.count, es};
-        else products[i] = tall ? OmxGemmProduct{x, cols, 1, a2, 1, r, xn, cols, run.rows, cols, cols, x, run.count, es}
+        else products[i] = tall ? OmxGemmProduct{x, cols, 1, a2, r, 1, xn, cols, run.rows, cols, cols, x, run.count, es}
                                 : OmxGemmProduct{a2, r, 1, x, cols, 1, xn, cols, r, r, c, x, run.count, es};
       }
       const int32_t rc = omx_gemm_frag32_group(ctx, products, count, stage < 2, stage == 1 ? s.b : s.a, stage == 1 ? s.c : 1.0f, omx_tag(ctx, F_MUON));
