@@ -338,6 +338,7 @@ int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);
 // f32 kernels: small outputs (gemm_frag32.hip) and direct-to-LDS loads (gemm_dma32.hip; g.K counts whole 32-column steps).
 // `_us`: what a tile is estimated to take; negative: not one for it.
 constexpr int FRAG32_TILES = 5, DMA32_TILES = 4;
+constexpr int FRAG32_EIGHT_WAVES = 4;  // tiles below this one share K between eight waves: the same sums in all
 // x: A k-contiguous, B k-major; w: both k-major. Estimate of a call of both (< 0: the tile does not fit), launch.
 constexpr int FRAG32_PAIRS = 4;
 double omx_gemm_frag32_pair_us(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w, int tile);

@@ -227,15 +227,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
 // ---- a linear layer's two gradients in one launch ----
 // A layer some hundred wide gives each of its two gradients less than a workgroup per compute unit or little more, and a call of the
 // two a fixed part of some 3 us twice and two part-empty rounds: their tiles go out together. w: both operands k-major, usually the
-// longer walk, so its workgroups come first; x: behind them, from workgroup `x_first` (a multiple of 8). Sums fold every 16 values
-// (frag32_sums): chains no longer than those of the kernels the two would take. A call of both with its host part: 1024 rows,
-// 256 -> 256 11.1 -> 7.1 us, 256 -> 704 17.3 -> 14.1, 704 -> 256 18.2 -> 13.7, 256 -> 128 10.3 -> 6.4; bound as gemm_frag32_kernel.
+// longer walk, so its workgroups come first; x: behind them, from workgroup `x_first` (a multiple of 8). x's sums are those of gemm_frag32_kernel's eight waves, whatever the tile: an
+// input gradient's bits are the same from a call that asks for it alone. w's fold every 16 values (frag32_sums). A call of both with
+// its host part: 1024 rows, 256 -> 256 11.1 -> 7.1 us, 256 -> 128 10.3 -> 6.4, 256 -> 12 9.5 -> 6.0; bound as gemm_frag32_kernel.
 constexpr int PAIR_WAVES = 8;
 template <int XM, int XN, int WM, int WN>
 __global__ __launch_bounds__(PAIR_WAVES * 64) void gemm_frag32_pair_kernel(GemmArgs x, GemmArgs w, int x_first) {
   extern __shared__ __attribute__((aligned(16))) float sums[];
   const int index = blockIdx.x;
-  if (index >= x_first) frag32_tile<false, true, XM, XN, PAIR_WAVES, true>(x, index - x_first, sums);
+  if (index >= x_first) frag32_tile<false, true, XM, XN, PAIR_WAVES, false>(x, index - x_first, sums);
   else if (index < w.tiles_m * w.tiles_n) frag32_tile<true, true, WM, WN, PAIR_WAVES, true>(w, index, sums);
 }
 

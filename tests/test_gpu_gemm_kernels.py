@@ -724,6 +724,8 @@ def test_both_gradients_in_one_launch(be, pair, rows, kin, nout):
     try:
         for got, want, bound in zip(be.linear_backward(dx, dw, dg), (g64 @ w64, g64.T @ x64), bounds):
             assert (np.abs(be.download(got) - want) <= bound + 1e-30).all()
+        if pair < 0:  # the input gradient's bits do not depend on who asks for it
+            assert np.array_equal(be.download(be.linear_backward(dx, dw, dg)[0]), be.download(be.linear_backward_input(dw, dg)))
         before = r.normal(size=x.shape).astype(np.float32)
         onto, gw = be.linear_backward_onto(be.upload(before), dx, dw, dg)
         assert (np.abs(be.download(onto) - (g64 @ w64 + before)) <= bounds[0] * (nout + 2) / (nout + 1) + 2.0 ** -23 * np.abs(before)).all()
