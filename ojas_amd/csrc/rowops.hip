@@ -16,13 +16,29 @@ constexpr int ROW_THREADS = 256;  // 4 waves per block, one row per wave at a ti
 // PER = ceil(dim / 64): lane l owns columns l, l + 64, ... so a wave's loads
 // are contiguous 64-element runs and the row stays in registers between the
 // sum-of-squares pass and the scaling pass.
+// One tensor, or two (queries and keys) side by side in the grid's second axis: apart they are two launches of 3 to 4 us, and two more
+// for their column sums, whatever their size.
+struct RmsRows {
+  const void *x, *gy;
+  const float* w;
+  void* y;         // the normed rows, or gx
+  float* partial;  // backward: [blocks][dim]
+  size_t rows;
+  int rows_per_block;
+  unsigned long long tag;
+};
+struct RmsTensors {
+  RmsRows of[2];
+};
 template <typename TX, typename TY, int PER>
-__global__ __launch_bounds__(ROW_THREADS) void rms_fwd_kernel(const TX* __restrict__ x, const float* __restrict__ w,
-                                                              TY* __restrict__ y, size_t rows, int dim, float eps,
-                                                              OmxFaultWord* fault, unsigned long long tag) {
+__global__ __launch_bounds__(ROW_THREADS) void rms_fwd_kernel(RmsTensors tensors, int dim, float eps, OmxFaultWord* fault) {
+  const RmsRows& t = tensors.of[blockIdx.y];
+  const TX* __restrict__ x = static_cast<const TX*>(t.x);
+  const float* __restrict__ w = t.w;
+  TY* __restrict__ y = static_cast<TY*>(t.y);
   const int lane = threadIdx.x & 63;
   const size_t row = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  if (row >= t.rows) return;
   const TX* xr = x + row * dim;
   float xv[PER];
   float ss = 0.0f;
@@ -46,18 +62,23 @@ __global__ __launch_bounds__(ROW_THREADS) void rms_fwd_kernel(const TX* __restri
       dev_store<TY>(yr, c, v);
     }
   }
-  if (bad) dev_raise_fault(fault, tag);
+  if (bad) dev_raise_fault(fault, t.tag);
 }
 
 // Backward: gx per row, and per-block partial column sums of g * xhat that a
 // second kernel adds in ascending block order (no atomics, deterministic).
 template <typename TX, typename TG, typename TO, int PER>
-__global__ __launch_bounds__(ROW_THREADS) void rms_bwd_kernel(const TX* __restrict__ x, const float* __restrict__ w,
-                                                              const TG* __restrict__ gy, TO* __restrict__ gx,
-                                                              float* __restrict__ partial, size_t rows, int dim,
-                                                              float eps, int rows_per_block, OmxFaultWord* fault,
-                                                              unsigned long long tag) {
+__global__ __launch_bounds__(ROW_THREADS) void rms_bwd_kernel(RmsTensors tensors, int dim, float eps, OmxFaultWord* fault) {
   extern __shared__ float lds[];  // [4][dim]
+  const RmsRows& t = tensors.of[blockIdx.y];
+  const TX* __restrict__ x = static_cast<const TX*>(t.x);
+  const float* __restrict__ w = t.w;
+  const TG* __restrict__ gy = static_cast<const TG*>(t.gy);
+  TO* __restrict__ gx = static_cast<TO*>(t.y);
+  float* __restrict__ partial = t.partial;
+  const size_t rows = t.rows;
+  const int rows_per_block = t.rows_per_block;
+  if (static_cast<size_t>(blockIdx.x) * rows_per_block >= rows) return;  // (the whole workgroup)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float inv_dim = 1.0f / static_cast<float>(dim);
   float wv[PER], accw[PER];
@@ -130,7 +151,7 @@ __global__ __launch_bounds__(ROW_THREADS) void rms_bwd_kernel(const TX* __restri
     float s = ((lds[c] + lds[dim + c]) + lds[2 * dim + c]) + lds[3 * dim + c];
     partial[static_cast<size_t>(blockIdx.x) * dim + c] = s;
   }
-  if (bad) dev_raise_fault(fault, tag);
+  if (bad) dev_raise_fault(fault, t.tag);
 }
 
 // out[c] = sum over blocks of partial[b][c]: 64 columns per workgroup, four
@@ -693,16 +714,13 @@ inline int per_for_dim(uint64_t dim) {
 }
 
 template <typename TX, typename TY>
-int32_t launch_rms_fwd(omx_ctx* ctx, const void* x, const float* w, void* y, uint64_t rows, uint64_t dim, float eps,
-                       unsigned long long tag) {
-  dim3 grid(static_cast<unsigned>((rows + 3) / 4)), block(ROW_THREADS);
-  int per = per_for_dim(dim);
-#define RMS_FWD(P)                                                                                              \
-  case P:                                                                                                       \
-    omx_launch(ctx, (rms_fwd_kernel<TX, TY, P>), grid, block, 0, static_cast<const TX*>(x), w, \
-                       static_cast<TY*>(y), rows, static_cast<int>(dim), eps, ctx->fault, tag);                 \
+int32_t launch_rms_fwd(omx_ctx* ctx, const RmsTensors& t, int count, uint64_t dim, float eps) {
+  const dim3 grid(static_cast<unsigned>((std::max(t.of[0].rows, t.of[1].rows) + 3) / 4), count), block(ROW_THREADS);
+#define RMS_FWD(P)                                                                                                   \
+  case P:                                                                                                            \
+    omx_launch(ctx, (rms_fwd_kernel<TX, TY, P>), grid, block, 0, t, static_cast<int>(dim), eps, ctx->fault);         \
     break;
-  switch (per) {
+  switch (per_for_dim(dim)) {
     RMS_FWD(1) RMS_FWD(2) RMS_FWD(4) RMS_FWD(8) RMS_FWD(12) RMS_FWD(16) RMS_FWD(32) RMS_FWD(64) RMS_FWD(128)
     default:
       return omx_fail(ctx, OMX_UNSUPPORTED, "rms_norm_forward: dim %llu above 8192", (unsigned long long)dim);
@@ -711,39 +729,62 @@ int32_t launch_rms_fwd(omx_ctx* ctx, const void* x, const float* w, void* y, uin
   OMX_LAUNCH_CHECK(ctx, "rms_fwd_kernel");
   return OMX_OK;
 }
+int32_t launch_rms_fwd(omx_ctx* ctx, const RmsTensors& t, int count, int32_t x_dtype, int32_t y_dtype, uint64_t dim, float eps) {
+  if (x_dtype == OMX_F32 && y_dtype == OMX_F32) return launch_rms_fwd<float, float>(ctx, t, count, dim, eps);
+  if (x_dtype == OMX_F32) return launch_rms_fwd<float, unsigned short>(ctx, t, count, dim, eps);
+  if (y_dtype == OMX_F32) return launch_rms_fwd<unsigned short, float>(ctx, t, count, dim, eps);
+  return launch_rms_fwd<unsigned short, unsigned short>(ctx, t, count, dim, eps);
+}
+
+// 32 rows per block, 16 where those are under a block per compute unit and there is room for as many partial rows, more when that
+// would leave over 2048 partial rows to add.
+uint64_t rms_partial_bytes(uint64_t blocks, uint64_t dim) { return (blocks + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float); }
+int rms_rows_per_block(omx_ctx* ctx, uint64_t rows, uint64_t dim) {
+  int rows_per_block = rows < 32ull * 256 && omx_workspace_fits(ctx, rms_partial_bytes((rows + 15) / 16, dim)) ? 16 : 32;
+  while ((rows + rows_per_block - 1) / rows_per_block > 2048 && rows_per_block < (1 << 20)) rows_per_block *= 2;
+  return rows_per_block;
+}
+uint64_t rms_blocks(const RmsRows& t) { return (t.rows + t.rows_per_block - 1) / t.rows_per_block; }
 
 template <typename TX, typename TG, typename TO>
-int32_t launch_rms_bwd(omx_ctx* ctx, const void* x, const float* w, const void* gy, void* gx, float* gw,
-                       uint64_t rows, uint64_t dim, float eps, unsigned long long tag) {
-  // 32 rows per block, 16 where those are under a block per compute unit and there is room for as many partial rows, more when that
-  // would leave over 2048 partial rows to add.
-  auto bytes_of = [&](uint64_t blocks) { return (blocks + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float); };
-  int rows_per_block = rows < 32ull * 256 && omx_workspace_fits(ctx, bytes_of((rows + 15) / 16)) ? 16 : 32;
-  while ((rows + rows_per_block - 1) / rows_per_block > 2048 && rows_per_block < (1 << 20)) rows_per_block *= 2;
-  uint64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
-  void* partial = nullptr;
-  int32_t rc = omx_workspace(ctx, bytes_of(blocks), &partial);
-  if (rc != OMX_OK) return rc;
-  // A narrow row leaves the column sum one or two workgroups: it then adds its rows in two stages.
-  float* stage = static_cast<float*>(partial) + blocks * dim;
-  dim3 grid(static_cast<unsigned>(blocks)), block(ROW_THREADS);
+int32_t launch_rms_bwd(omx_ctx* ctx, const RmsTensors& t, int count, uint64_t dim, float eps) {
+  const uint64_t blocks = count == 1 ? rms_blocks(t.of[0]) : std::max(rms_blocks(t.of[0]), rms_blocks(t.of[1]));
+  dim3 grid(static_cast<unsigned>(blocks), count), block(ROW_THREADS);
   size_t smem = 4 * dim * sizeof(float);
-  int per = per_for_dim(dim);
-#define RMS_BWD(P)                                                                                                  \
-  case P:                                                                                                           \
-    omx_launch(ctx, (rms_bwd_kernel<TX, TG, TO, P>), grid, block, smem, static_cast<const TX*>(x), \
-                       w, static_cast<const TG*>(gy), static_cast<TO*>(gx), static_cast<float*>(partial), rows,     \
-                       static_cast<int>(dim), eps, rows_per_block, ctx->fault, tag);                                \
+#define RMS_BWD(P)                                                                                                   \
+  case P:                                                                                                            \
+    omx_launch(ctx, (rms_bwd_kernel<TX, TG, TO, P>), grid, block, smem, t, static_cast<int>(dim), eps, ctx->fault);  \
     break;
-  switch (per) {
+  switch (per_for_dim(dim)) {
     RMS_BWD(1) RMS_BWD(2) RMS_BWD(4) RMS_BWD(8) RMS_BWD(12) RMS_BWD(16) RMS_BWD(32) RMS_BWD(64)
     default:
       return omx_fail(ctx, OMX_UNSUPPORTED, "rms_norm_backward: dim %llu above 4096", (unsigned long long)dim);
   }
 #undef RMS_BWD
   OMX_LAUNCH_CHECK(ctx, "rms_bwd_kernel");
-  return omx_column_sum(ctx, static_cast<const float*>(partial), gw, blocks, dim, tag, stage);
+  return OMX_OK;
 }
+int32_t launch_rms_bwd(omx_ctx* ctx, const RmsTensors& t, int count, int32_t x_dtype, int32_t gy_dtype, int32_t gx_dtype, uint64_t dim,
+                       float eps) {
+  typedef unsigned short h16;
+  switch ((x_dtype == OMX_BF16 ? 4 : 0) | (gy_dtype == OMX_BF16 ? 2 : 0) | (gx_dtype == OMX_BF16 ? 1 : 0)) {
+    case 0: return launch_rms_bwd<float, float, float>(ctx, t, count, dim, eps);
+    case 1: return launch_rms_bwd<float, float, h16>(ctx, t, count, dim, eps);
+    case 2: return launch_rms_bwd<float, h16, float>(ctx, t, count, dim, eps);
+    case 3: return launch_rms_bwd<float, h16, h16>(ctx, t, count, dim, eps);
+    case 4: return launch_rms_bwd<h16, float, float>(ctx, t, count, dim, eps);
+    case 5: return launch_rms_bwd<h16, float, h16>(ctx, t, count, dim, eps);
+    case 6: return launch_rms_bwd<h16, h16, float>(ctx, t, count, dim, eps);
+    default: return launch_rms_bwd<h16, h16, h16>(ctx, t, count, dim, eps);
+  }
+}
+
+// Whether two ranges share no byte.
+bool no_overlap(const void* a, uint64_t a_bytes, const void* b, uint64_t b_bytes) {
+  const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+  return pa + a_bytes <= pb || pb + b_bytes <= pa;
+}
+uint64_t float_bytes(int32_t dtype) { return dtype == OMX_BF16 ? 2 : 4; }
 
 int32_t rms_forward_impl(omx_ctx* ctx, const char* op, uint32_t fault_op, const void* x, int32_t x_dtype,
                          const void* w, void* y, int32_t y_dtype, uint64_t rows, uint64_t dim, float eps) {
@@ -752,10 +793,9 @@ int32_t rms_forward_impl(omx_ctx* ctx, const char* op, uint32_t fault_op, const 
   const float* wf = static_cast<const float*>(w);
   if (omx_rms_vec_eligible(dim, {x, w, y}))
     return omx_rms_forward_vec(ctx, x, x_dtype, nullptr, OMX_F32, wf, nullptr, y, y_dtype, rows, dim, eps, tag);
-  if (x_dtype == OMX_F32 && y_dtype == OMX_F32) return launch_rms_fwd<float, float>(ctx, x, wf, y, rows, dim, eps, tag);
-  if (x_dtype == OMX_F32) return launch_rms_fwd<float, unsigned short>(ctx, x, wf, y, rows, dim, eps, tag);
-  if (y_dtype == OMX_F32) return launch_rms_fwd<unsigned short, float>(ctx, x, wf, y, rows, dim, eps, tag);
-  return launch_rms_fwd<unsigned short, unsigned short>(ctx, x, wf, y, rows, dim, eps, tag);
+  RmsTensors t{};
+  t.of[0] = {x, nullptr, wf, y, nullptr, rows, 0, tag};
+  return launch_rms_fwd(ctx, t, 1, x_dtype, y_dtype, dim, eps);
 }
 
 int32_t rms_backward_impl(omx_ctx* ctx, uint32_t fault_op, const void* x, int32_t x_dtype, const void* w,
@@ -767,18 +807,17 @@ int32_t rms_backward_impl(omx_ctx* ctx, uint32_t fault_op, const void* x, int32_
   if (omx_rms_vec_eligible(dim, {x, w, gy, gx, gw}))
     return omx_rms_backward_vec(ctx, x, x_dtype, wf, gy, gy_dtype, nullptr, gx, gx_dtype, nullptr, gwf, rows, dim, eps,
                                 tag);
-  typedef unsigned short h16;
-  const int key = (x_dtype == OMX_BF16 ? 4 : 0) | (gy_dtype == OMX_BF16 ? 2 : 0) | (gx_dtype == OMX_BF16 ? 1 : 0);
-  switch (key) {
-    case 0: return launch_rms_bwd<float, float, float>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-    case 1: return launch_rms_bwd<float, float, h16>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-    case 2: return launch_rms_bwd<float, h16, float>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-    case 3: return launch_rms_bwd<float, h16, h16>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-    case 4: return launch_rms_bwd<h16, float, float>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-    case 5: return launch_rms_bwd<h16, float, h16>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-    case 6: return launch_rms_bwd<h16, h16, float>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-    default: return launch_rms_bwd<h16, h16, h16>(ctx, x, wf, gy, gx, gwf, rows, dim, eps, tag);
-  }
+  RmsTensors t{};
+  t.of[0] = {x, gy, wf, gx, nullptr, rows, rms_rows_per_block(ctx, rows, dim), tag};
+  const uint64_t blocks = rms_blocks(t.of[0]);
+  void* partial = nullptr;
+  int32_t rc = omx_workspace(ctx, rms_partial_bytes(blocks, dim), &partial);
+  if (rc != OMX_OK) return rc;
+  t.of[0].partial = static_cast<float*>(partial);
+  rc = launch_rms_bwd(ctx, t, 1, x_dtype, gy_dtype, gx_dtype, dim, eps);
+  if (rc != OMX_OK) return rc;
+  // A narrow row leaves the column sum one or two workgroups: it then adds its rows in two stages.
+  return omx_column_sum(ctx, t.of[0].partial, gwf, blocks, dim, tag, t.of[0].partial + blocks * dim);
 }
 
 bool finite_host(float v) { return v == v && v != INFINITY && v != -INFINITY; }
@@ -910,6 +949,16 @@ int32_t omx_rms_qk_norm_forward(omx_ctx* ctx, const void* q, const void* k, int3
     return omx_fail(ctx, OMX_DTYPE, "%s: dtype must be f32 or bf16", op);
   if (q_rows == 0 || k_rows == 0 || dim == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
   if (!finite_host(eps)) return omx_fail(ctx, OMX_NON_FINITE, "%s", op);
+  const uint64_t in = float_bytes(x_dtype) * dim, out = float_bytes(y_dtype) * dim;
+  if (!omx_rms_vec_eligible(dim, {q, q_weight, q_out}) && !omx_rms_vec_eligible(dim, {k, k_weight, k_out}) &&
+      no_overlap(q_out, q_rows * out, k, k_rows * in) && no_overlap(q_out, q_rows * out, k_weight, dim * 4) &&
+      no_overlap(k_out, k_rows * out, q, q_rows * in) && no_overlap(k_out, k_rows * out, q_weight, dim * 4) &&
+      no_overlap(q_out, q_rows * out, k_out, k_rows * out)) {
+    RmsTensors t{};
+    t.of[0] = {q, nullptr, static_cast<const float*>(q_weight), q_out, nullptr, q_rows, 0, omx_tag(ctx, F_RMS_QK_FORWARD)};
+    t.of[1] = {k, nullptr, static_cast<const float*>(k_weight), k_out, nullptr, k_rows, 0, omx_tag(ctx, F_RMS_QK_FORWARD)};
+    return launch_rms_fwd(ctx, t, 2, x_dtype, y_dtype, dim, eps);
+  }
   int32_t rc = rms_forward_impl(ctx, op, F_RMS_QK_FORWARD, q, x_dtype, q_weight, q_out, y_dtype, q_rows, dim, eps);
   if (rc != OMX_OK) return rc;
   return rms_forward_impl(ctx, op, F_RMS_QK_FORWARD, k, x_dtype, k_weight, k_out, y_dtype, k_rows, dim, eps);
@@ -927,6 +976,46 @@ int32_t omx_rms_qk_norm_backward(omx_ctx* ctx, const void* q, const void* k, int
     return omx_fail(ctx, OMX_DTYPE, "%s: dtype must be f32 or bf16", op);
   if (q_rows == 0 || k_rows == 0 || dim == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
   if (!finite_host(eps)) return omx_fail(ctx, OMX_NON_FINITE, "%s", op);
+  const uint64_t in = float_bytes(x_dtype) * dim, grad = float_bytes(gy_dtype) * dim, out = float_bytes(gx_dtype) * dim;
+  bool together = !omx_rms_vec_eligible(dim, {q, q_weight, grad_q, gq, gq_weight}) && !omx_rms_vec_eligible(dim, {k, k_weight, grad_k, gk, gk_weight}) &&
+                  no_overlap(gq, q_rows * out, gk, k_rows * out);
+  struct Range {
+    const void* at;
+    uint64_t bytes;
+  };
+  const Range of_q[] = {{q, q_rows * in}, {q_weight, dim * 4}, {grad_q, q_rows * grad}, {gq_weight, dim * 4}};
+  const Range of_k[] = {{k, k_rows * in}, {k_weight, dim * 4}, {grad_k, k_rows * grad}, {gk_weight, dim * 4}};
+  for (const Range& r : of_k) together = together && no_overlap(gq, q_rows * out, r.at, r.bytes) && no_overlap(gq_weight, dim * 4, r.at, r.bytes);
+  for (const Range& r : of_q) together = together && no_overlap(gk, k_rows * out, r.at, r.bytes) && no_overlap(gk_weight, dim * 4, r.at, r.bytes);
+  if (together) {
+    RmsTensors t{};
+    t.of[0] = {q, grad_q, static_cast<const float*>(q_weight), gq, nullptr, q_rows, rms_rows_per_block(ctx, q_rows, dim), 0};
+    t.of[1] = {k, grad_k, static_cast<const float*>(k_weight), gk, nullptr, k_rows, rms_rows_per_block(ctx, k_rows, dim), 0};
+    const uint64_t blocks[2] = {rms_blocks(t.of[0]), rms_blocks(t.of[1])};
+    const uint64_t q_bytes = (rms_partial_bytes(blocks[0], dim) + 255) / 256 * 256, bytes = q_bytes + rms_partial_bytes(blocks[1], dim);
+    void* partial = omx_workspace_if_room(ctx, bytes);
+    if (partial) {
+      float* const weights[2] = {static_cast<float*>(gq_weight), static_cast<float*>(gk_weight)};
+      bool wide = true;
+      for (int i = 0; i < 2; ++i) {
+        t.of[i].partial = reinterpret_cast<float*>(static_cast<char*>(partial) + i * q_bytes);
+        t.of[i].tag = omx_tag(ctx, F_RMS_QK_BACKWARD);
+        wide = wide && blocks[i] > 16 && blocks[i] <= OMX_COLUMN_SUM_WIDE_ROWS;
+      }
+      int32_t rc = launch_rms_bwd(ctx, t, 2, x_dtype, gy_dtype, gx_dtype, dim, eps);
+      if (rc != OMX_OK) return rc;
+      if (wide) {
+        ColumnSumList list{};
+        for (int i = 0; i < 2; ++i) list.of[i] = {t.of[i].partial, weights[i], t.of[i].tag, static_cast<int>(blocks[i]), static_cast<int>(dim)};
+        omx_launch(ctx, column_sum_list_kernel, dim3(static_cast<unsigned>((dim + 63) / 64), 2), dim3(1024), 0, list, ctx->fault);
+        OMX_LAUNCH_CHECK(ctx, "column_sum_list_kernel");
+        return OMX_OK;
+      }
+      for (int i = 0; i < 2 && rc == OMX_OK; ++i)
+        rc = omx_column_sum(ctx, t.of[i].partial, weights[i], blocks[i], dim, t.of[i].tag, t.of[i].partial + blocks[i] * dim);
+      return rc;
+    }
+  }
   int32_t rc = rms_backward_impl(ctx, F_RMS_QK_BACKWARD, q, x_dtype, q_weight, grad_q, gy_dtype, gq, gx_dtype,
                                  gq_weight, q_rows, dim, eps);
   if (rc != OMX_OK) return rc;

@@ -152,6 +152,35 @@ def test_rms_qk_norm(be, b, t, h, kvh, d, bf16):
     close(be.download_f32(got[3]), wk[1], wtol, "gk_weight")
 
 
+@pytest.mark.parametrize("b,t,h,kvh,d", [(1, 1, 1, 1, 4), (1, 3, 2, 1, 10), (2, 300, 4, 1, 64), (1, 600, 4, 2, 64), (3, 700, 4, 4, 32), (1, 40, 3, 3, 130)])
+def test_rms_qk_norm_carries_the_bits_of_two_norms(be, b, t, h, kvh, d):
+    """Queries and keys in one launch each way, and the two column sums where both add 17 partial rows and more; a value that is not
+    finite is named in either."""
+    from ojas_amd.backend import OjasError
+
+    print(f"rms_qk_norm together {b}x{t}x{h}/{kvh}x{d}", flush=True)
+    r = np.random.default_rng(b + t + d)
+    q, k, gq, gk = (r.standard_normal((b, t, n, d), dtype=np.float32) for n in (h, kvh, h, kvh))
+    qw, kw = (be.upload(r.standard_normal(d, dtype=np.float32)) for _ in range(2))
+    dq, dk, dgq, dgk = (be.upload(a) for a in (q, k, gq, gk))
+    for got, x, w in zip(be.rms_qk_norm_forward(dq, dk, qw, kw, 1e-6), (dq, dk), (qw, kw)):
+        assert np.array_equal(be.download(got), be.download(be.rms_norm_forward(x, w, 1e-6)))
+    got = be.rms_qk_norm_backward(dq, dk, qw, kw, dgq, dgk, 1e-6)
+    for i, (x, w, g) in enumerate(((dq, qw, dgq), (dk, kw, dgk))):
+        want = be.rms_norm_backward(x, w, g, 1e-6)
+        assert np.array_equal(be.download(got[i]), be.download(want[0])) and np.array_equal(be.download(got[2 + i]), be.download(want[1]))
+    for bad in (q, k):
+        held = bad[-1, -1, -1, -1]
+        bad[-1, -1, -1, -1] = np.nan
+        pair = be.upload(q), be.upload(k)
+        for call in (lambda: be.rms_qk_norm_forward(*pair, qw, kw, 1e-6), lambda: be.rms_qk_norm_backward(*pair, qw, kw, dgq, dgk, 1e-6)):
+            call()
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.detail.startswith("rms_qk_norm")
+        bad[-1, -1, -1, -1] = held
+
+
 GATE_SHAPES = [(1, 2, 2, 1), (37, 24, 3, 8), (257, 128, 12, 64), (64, 768, 12, 64), (19, 40, 5, 5), (130, 96, 6, 32)]
 
 
