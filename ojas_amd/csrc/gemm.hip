@@ -506,8 +506,10 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 }  // namespace
 
 // Both gradients of an f32 linear layer in one launch where that is estimated to take less (259 layers of
-// 24 .. 6000 rows and 12 .. 1600 columns: 4.44 -> 3.80 ms of calls in all, the three it lost on 5, 6 and 12 % slower). onto: gx is
-// added to. False: not taken.
+// 24 .. 6000 rows and 12 .. 1600 columns: 4.44 -> 3.80 ms of calls in all, the three it lost on 5, 6 and 12 % slower; 157 of whole
+// steps, where gx takes the direct-to-LDS form: 4.13 -> 3.66, one 8 % slower). gx has the bits of a call that asks for it alone: the
+// form is the one of f32_tile's choice for it, with the estimate of the 32 x 32 pair for the direct-to-LDS ones (at 1.1 and 1.25
+// of the two apart, 5 and 11 of the 157 lost). onto: gx is added to. False: not taken.
 bool omx_linear_backward_pair(omx_ctx* ctx, const float* x, const float* w, const float* gy, float* gx, float* gw, uint64_t rows, uint64_t in,
                               uint64_t out, bool onto, int32_t* rc) {
   const uint64_t most = 0x7fffffff;
@@ -544,28 +546,27 @@ bool omx_linear_backward_pair(omx_ctx* ctx, const float* x, const float* w, cons
   gemm_w.K = gemm_w.k_rows = gemm_w.a_k = static_cast<int>(rows);
   gemm_w.b_vec = aligned16(x) && in % 4 == 0;
   gemm_w.c_vec = aligned16(gw) && in % 4 == 0;
+  int frag32 = -1, dma32 = -1;
+  const double x_us = f32_tile(ctx, gemm_x, false, true, &frag32, &dma32);
   int tile = -1;
   double best = 1e30;
   for (int t = 0; t < FRAG32_PAIRS; ++t) {
     const double us = ctx->gemm_f32_pair < 0 || ctx->gemm_f32_pair == t + 1 ? omx_gemm_frag32_pair_us(ctx, gemm_x, gemm_w, t) : -1.0;
-    if (us >= 0.0 && us < best) {
+    if (us >= 0.0 && us < best && (dma32 < 0 || ctx->gemm_f32_pair > 0 || t == 2)) {
       best = us;
       tile = t;
     }
   }
   if (tile < 0) return false;
   if (ctx->gemm_f32_pair < 0) {
-    int frag32 = -1, dma32 = -1;
-    double two = f32_tile(ctx, gemm_x, false, true, &frag32, &dma32);
-    if (frag32 < 0 || frag32 >= FRAG32_EIGHT_WAVES) return false;  // (a call for gx alone would sum in another order)
-    frag32 = dma32 = -1;
-    two += f32_tile(ctx, gemm_w, true, true, &frag32, &dma32);
-    if (best > two) return false;
+    int w_frag32 = -1, w_dma32 = -1;
+    if (dma32 < 0 && (frag32 < 0 || frag32 >= FRAG32_EIGHT_WAVES)) return false;  // (a call for gx alone would sum in another order)
+    if (best > x_us + f32_tile(ctx, gemm_w, true, true, &w_frag32, &w_dma32)) return false;
   }
   gemm_w.tag = gemm_w.act_tag = omx_tag(ctx, F_LINEAR_BACKWARD);
   gemm_x.accumulate = onto;
   gemm_x.tag = gemm_x.act_tag = onto ? omx_tag(ctx, F_GEMM) : gemm_w.tag;  // (named as the two calls it stands for)
-  *rc = omx_gemm_frag32_pair(ctx, gemm_x, gemm_w, tile);
+  *rc = ctx->gemm_f32_pair < 0 && dma32 >= 0 ? omx_gemm_dma32_pair(ctx, gemm_x, gemm_w, dma32) : omx_gemm_frag32_pair(ctx, gemm_x, gemm_w, tile);
   return true;
 }
 

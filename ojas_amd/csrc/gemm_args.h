@@ -343,6 +343,7 @@ constexpr int FRAG32_EIGHT_WAVES = 4;  // tiles below this one share K between e
 constexpr int FRAG32_PAIRS = 4;
 double omx_gemm_frag32_pair_us(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w, int tile);
 int32_t omx_gemm_frag32_pair(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w, int tile);
+int32_t omx_gemm_dma32_pair(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w, int dma32);
 double omx_gemm_frag32_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
 int32_t omx_gemm_frag32_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int tile);
 // Independent f32 products C = A.B, or s1 aux + s2 A.B where `aux` is set (C's layout), in one launch; strides in elements, as

@@ -239,6 +239,22 @@ __global__ __launch_bounds__(PAIR_WAVES * 64) void gemm_frag32_pair_kernel(GemmA
   else if (index < w.tiles_m * w.tiles_n) frag32_tile<true, true, WM, WN, PAIR_WAVES, true>(w, index, sums);
 }
 
+// The same where the input gradient alone would run on gemm_dma32_kernel with KG groups of waves: its sums, on eight waves. 1024 rows,
+// 256 -> 704 16.7 -> 13.2 us a call, 704 -> 256 18.2 -> 14.4; 512 rows of 512 -> 512 13.0 -> 9.9.
+template <int KG>
+struct PairDma;  // waves of a group, blocks of a wave
+template <> struct PairDma<1> { static constexpr int WGM = 4, WGN = 2, TM = 1, TN = 2; };
+template <> struct PairDma<2> { static constexpr int WGM = 2, WGN = 2, TM = 2, TN = 1; };
+template <> struct PairDma<4> { static constexpr int WGM = 1, WGN = 2, TM = 2, TN = 1; };
+template <int KG>
+__global__ __launch_bounds__(PAIR_WAVES * 64) void gemm_dma32_pair_kernel(GemmArgs x, GemmArgs w, int x_first) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  using D = PairDma<KG>;
+  const int index = blockIdx.x;
+  if (index >= x_first) dma32_tile<false, true, D::WGM, D::WGN, D::TM, D::TN, 2, KG, false, 0>(x, index - x_first, smem);
+  else if (index < w.tiles_m * w.tiles_n) frag32_tile<true, true, 2, 2, PAIR_WAVES, true>(w, index, reinterpret_cast<float*>(smem));
+}
+
 // ---- several products in one launch ----
 // Five shapes of a model's matrices are five chains of fifteen Newton-Schulz products, each a launch of 4 to 256 workgroups that takes
 // 3 to 13 us and leaves most of the chip idle: the k-th products of all chains go out together. 32 x 32 tiles whose four waves share
@@ -417,6 +433,21 @@ int32_t launch_pair(omx_ctx* ctx, GemmArgs x, GemmArgs w) {
 // over 326 layers of 24 .. 6000 rows and 12 .. 1600 columns, each on all four pairs (rms 7 %); the tiles it chooses are 1.4 % behind
 // the best of the four on average (32 x 32 for both 17 %).
 namespace {
+template <int KG>
+int32_t launch_dma_pair(omx_ctx* ctx, GemmArgs x, GemmArgs w) {
+  using D = PairDma<KG>;
+  constexpr int BM = D::WGM * D::TM * 16, BN = D::WGN * D::TN * 16;
+  constexpr int smem = std::max(2 * KG * (BM + BN) * 128, PAIR_WAVES * 32 * 36 * 4);
+  static_assert(smem <= 64 * 1024 && D::WGM * D::WGN * KG == PAIR_WAVES, "what a launch may ask for");
+  x.tiles_m = (x.M + BM - 1) / BM;
+  x.tiles_n = (x.N + BN - 1) / BN;
+  w.tiles_m = (w.M + 31) / 32;
+  w.tiles_n = (w.N + 31) / 32;
+  const int x_first = (w.tiles_m * w.tiles_n + 7) & ~7;
+  omx_launch(ctx, (gemm_dma32_pair_kernel<KG>), dim3(static_cast<unsigned>(x_first + x.tiles_m * x.tiles_n)), dim3(PAIR_WAVES * 64), smem, x, w, x_first);
+  OMX_LAUNCH_CHECK(ctx, "gemm_dma32_pair_kernel");
+  return OMX_OK;
+}
 constexpr double PAIR_US = 2.83;
 struct PairTile {
   int xm, xn, wm, wn;
@@ -455,6 +486,10 @@ int32_t omx_gemm_frag32_pair(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w,
     case 2: return launch_pair_tile<2>(ctx, x, w);
     default: return launch_pair_tile<3>(ctx, x, w);
   }
+}
+int32_t omx_gemm_dma32_pair(omx_ctx* ctx, const GemmArgs& x, const GemmArgs& w, int dma32) {
+  if (dma32 < 2) return launch_dma_pair<1>(ctx, x, w);
+  return dma32 == 2 ? launch_dma_pair<2>(ctx, x, w) : launch_dma_pair<4>(ctx, x, w);
 }
 
 // (The operands are the library's own scratch: what does not fit is a mistake of the caller's.)

@@ -706,7 +706,8 @@ def test_f32_activation_in_the_store_pass_is_named_as_the_separate_pass_is(be, t
 
 
 @pytest.mark.parametrize("pair", [1, 2, 3, 4, -1])
-@pytest.mark.parametrize("rows,kin,nout", [(1, 4, 4), (16, 32, 16), (65, 34, 20), (130, 96, 36), (257, 70, 12), (1021, 66, 132), (300, 512, 260), (4100, 32, 64)])
+@pytest.mark.parametrize("rows,kin,nout", [(1, 4, 4), (16, 32, 16), (65, 34, 20), (130, 96, 36), (257, 70, 12), (1021, 66, 132), (300, 512, 260), (4100, 32, 64),
+                                           (700, 900, 256), (900, 516, 320), (500, 380, 512)])  # last: gx on 1, 2 and 4 groups of waves
 def test_both_gradients_in_one_launch(be, pair, rows, kin, nout):
     """Each pair of tiles, forced where it fits, and the rule's choice: outputs that end inside a tile, walks of one step, of fewer
     steps than waves and ending inside one, more tiles than compute units; against the f64 products, k products and k sums rounded
