@@ -538,6 +538,11 @@ int32_t omx_mul_forward(omx_ctx* ctx, const void* a, const void* b, void* out, i
                         uint64_t n);
 int32_t omx_mul_backward(omx_ctx* ctx, const void* a, const void* b, const void* gy, void* ga,
                          void* gb, int32_t dtype, uint64_t n);
+/* out = silu(gate) up and its reverse, each pair of ops in one pass with the bits of the two (f32). The gradients are written apart
+ * from the operands. */
+int32_t omx_silu_mul_forward(omx_ctx* ctx, const void* gate, const void* up, void* out, uint64_t n);
+int32_t omx_silu_mul_backward(omx_ctx* ctx, const void* gate, const void* up, const void* gy, void* g_gate, void* g_up,
+                              uint64_t n);
 /* BackendModule::rope_half_split_forward / _backward (backend.rs:1674-1686; CPU
  * ojas-cpu/src/norm.rs:271-312). x is [rows, dim] with dim even; cos / sin are
  * f32. heads > 0: tables are [time, dim] and row r uses table row

@@ -140,6 +140,8 @@ extern "C" {
     pub fn omx_silu_backward(ctx: *mut OmxCtx, x: *const c_void, gy: *const c_void, gx: *mut c_void, dtype: i32, n: u64) -> i32;
     pub fn omx_mul_forward(ctx: *mut OmxCtx, a: *const c_void, b: *const c_void, out: *mut c_void, dtype: i32, n: u64) -> i32;
     pub fn omx_mul_backward(ctx: *mut OmxCtx, a: *const c_void, b: *const c_void, gy: *const c_void, ga: *mut c_void, gb: *mut c_void, dtype: i32, n: u64) -> i32;
+    pub fn omx_silu_mul_forward(ctx: *mut OmxCtx, gate: *const c_void, up: *const c_void, out: *mut c_void, n: u64) -> i32;
+    pub fn omx_silu_mul_backward(ctx: *mut OmxCtx, gate: *const c_void, up: *const c_void, gy: *const c_void, g_gate: *mut c_void, g_up: *mut c_void, n: u64) -> i32;
     pub fn omx_rope_half_split_forward(ctx: *mut OmxCtx, x: *const c_void, cos_f32: *const c_void, sin_f32: *const c_void, y: *mut c_void, dtype: i32, rows: u64, dim: u64, time: u64, heads: u64) -> i32;
     pub fn omx_rope_half_split_backward(ctx: *mut OmxCtx, gy: *const c_void, cos_f32: *const c_void, sin_f32: *const c_void, gx: *mut c_void, dtype: i32, rows: u64, dim: u64, time: u64, heads: u64) -> i32;
     pub fn omx_rope_half_split_inplace(ctx: *mut OmxCtx, x: *mut c_void, dtype: i32, pitch: u64, cos_f32: *const c_void, sin_f32: *const c_void, tokens: u64, time: u64, heads: u64, dim: u64, backward: i32) -> i32;

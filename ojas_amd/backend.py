@@ -776,6 +776,24 @@ class MiBackend(_native.Methods):
         _native.omx_mul_backward(self._context, a, b, gy, ga, gb, a.dtype, a.numel)
         return ga, gb
 
+    def silu_mul_forward(self, gate, up):
+        """`mul_forward(silu_forward(gate), up)` in one pass (f32)."""
+        self._same("silu_mul_forward", gate, up)
+        if gate.dtype != F32:
+            raise OjasError(DTYPE, "silu_mul_forward: f32 operands")
+        out = self.empty(gate.shape, F32)
+        _native.omx_silu_mul_forward(self._context, gate, up, out, gate.numel)
+        return out
+
+    def silu_mul_backward(self, gate, up, gy):
+        """Gradients of `silu_mul_forward` by gate and up."""
+        self._same("silu_mul_backward", gate, up, gy)
+        if gate.dtype != F32:
+            raise OjasError(DTYPE, "silu_mul_backward: f32 operands")
+        g_gate, g_up = self.empty(gate.shape, F32), self.empty(gate.shape, F32)
+        _native.omx_silu_mul_backward(self._context, gate, up, gy, g_gate, g_up, gate.numel)
+        return g_gate, g_up
+
     def _rope(self, fn, op, x, cos, sin):
         if cos.shape != sin.shape:
             raise OjasError(SHAPE, f"{op}: cos shape {cos.shape} != sin shape {sin.shape}")

@@ -104,6 +104,60 @@ __global__ __launch_bounds__(BK_THREADS) void mul_bwd_kernel(const T* __restrict
   if (bad) dev_raise_fault(fault, tag);
 }
 
+// silu(gate) * up and its reverse in one pass each, f32, with the bits of the two ops and their names for what is not finite. The
+// activation is formed again instead of kept. 1024 x 704: 2.6 + 3.1 -> 3.2 us and 3.9 + 3.6 -> 4.4; bound by a launch's latency
+// there, by memory (two reads and a write; three and two) above.
+template <typename T, int V>
+__global__ __launch_bounds__(BK_THREADS) void silu_mul_fwd_kernel(const T* __restrict__ gate, const T* __restrict__ up,
+                                                                  T* __restrict__ out, size_t packs, OmxFaultWord* fault,
+                                                                  unsigned long long silu_tag, unsigned long long mul_tag) {
+  bool bad_silu = false, bad_mul = false;
+  PACK_LOOP(p, packs) {
+    float v[V], y[V], r[V];
+    load_pack<T, V>(gate, p, v);
+    load_pack<T, V>(up, p, y);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      float s, rest;
+      sigmoid_pair(v[j], &s, &rest);
+      const float act = v[j] * s;
+      r[j] = act * y[j];
+      bad_silu |= !dev_finite(act);
+      bad_mul |= !dev_finite(r[j]);
+    }
+    store_pack<T, V>(out, p, r);
+  }
+  if (bad_silu) dev_raise_fault(fault, silu_tag);
+  if (bad_mul) dev_raise_fault(fault, mul_tag);
+}
+template <typename T, int V>
+__global__ __launch_bounds__(BK_THREADS) void silu_mul_bwd_kernel(const T* __restrict__ gate, const T* __restrict__ up,
+                                                                  const T* __restrict__ gy, T* __restrict__ g_gate,
+                                                                  T* __restrict__ g_up, size_t packs, OmxFaultWord* fault,
+                                                                  unsigned long long mul_tag, unsigned long long silu_tag) {
+  bool bad_silu = false, bad_mul = false;
+  PACK_LOOP(p, packs) {
+    float v[V], y[V], g[V], ra[V], rb[V];
+    load_pack<T, V>(gate, p, v);
+    load_pack<T, V>(up, p, y);
+    load_pack<T, V>(gy, p, g);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      float s, rest;
+      sigmoid_pair(v[j], &s, &rest);
+      const float g_act = g[j] * y[j];
+      rb[j] = g[j] * (v[j] * s);
+      ra[j] = g_act * s * (1.0f + v[j] * rest);
+      bad_mul |= !(dev_finite(g_act) && dev_finite(rb[j]));
+      bad_silu |= !dev_finite(ra[j]);
+    }
+    store_pack<T, V>(g_gate, p, ra);
+    store_pack<T, V>(g_up, p, rb);
+  }
+  if (bad_mul) dev_raise_fault(fault, mul_tag);
+  if (bad_silu) dev_raise_fault(fault, silu_tag);
+}
+
 // ------------------------------------------------------------------- RoPE
 // One thread owns V columns of the first half of a row and the matching V of
 // the second half. y = x cos + cat(-x2, x1) sin; the backward is its
@@ -527,6 +581,32 @@ int32_t omx_mul_backward(omx_ctx* ctx, const void* a, const void* b, const void*
   LAUNCH_TV(mul_bwd_kernel, dtype, vec, pack_grid(packs), static_cast<const T_*>(a), static_cast<const T_*>(b),
             static_cast<const T_*>(gy), static_cast<T_*>(ga), static_cast<T_*>(gb), packs, ctx->fault, tag);
   OMX_LAUNCH_CHECK(ctx, "mul_bwd_kernel");
+  return OMX_OK;
+}
+
+int32_t omx_silu_mul_forward(omx_ctx* ctx, const void* gate, const void* up, void* out, uint64_t n) {
+  OMX_REQUIRE_CTX(ctx);
+  const int32_t rc = check_unary(ctx, "silu_mul_forward", OMX_F32, n, {gate, up, out});
+  if (rc != OMX_OK) return rc;
+  const bool vec = packs_of_four(n, 4, {gate, up, out});
+  const size_t packs = vec ? n / 4 : n;
+  const unsigned long long silu_tag = omx_tag(ctx, F_SILU_FORWARD), mul_tag = omx_tag(ctx, F_MUL_FORWARD);
+  omx_launch(ctx, (vec ? &silu_mul_fwd_kernel<float, 4> : &silu_mul_fwd_kernel<float, 1>), pack_grid(packs), dim3(BK_THREADS), 0,
+             static_cast<const float*>(gate), static_cast<const float*>(up), static_cast<float*>(out), packs, ctx->fault, silu_tag, mul_tag);
+  OMX_LAUNCH_CHECK(ctx, "silu_mul_fwd_kernel");
+  return OMX_OK;
+}
+int32_t omx_silu_mul_backward(omx_ctx* ctx, const void* gate, const void* up, const void* gy, void* g_gate, void* g_up, uint64_t n) {
+  OMX_REQUIRE_CTX(ctx);
+  const int32_t rc = check_unary(ctx, "silu_mul_backward", OMX_F32, n, {gate, up, gy, g_gate, g_up});
+  if (rc != OMX_OK) return rc;
+  const bool vec = packs_of_four(n, 4, {gate, up, gy, g_gate, g_up});
+  const size_t packs = vec ? n / 4 : n;
+  const unsigned long long mul_tag = omx_tag(ctx, F_MUL_BACKWARD), silu_tag = omx_tag(ctx, F_SILU_BACKWARD);
+  omx_launch(ctx, (vec ? &silu_mul_bwd_kernel<float, 4> : &silu_mul_bwd_kernel<float, 1>), pack_grid(packs), dim3(BK_THREADS), 0,
+             static_cast<const float*>(gate), static_cast<const float*>(up), static_cast<const float*>(gy), static_cast<float*>(g_gate),
+             static_cast<float*>(g_up), packs, ctx->fault, mul_tag, silu_tag);
+  OMX_LAUNCH_CHECK(ctx, "silu_mul_bwd_kernel");
   return OMX_OK;
 }
 

@@ -467,7 +467,7 @@ struct Symbol {
   X(omx_embedding_backward_accumulate) X(omx_adamw_step) X(omx_adamw_step_bounded) X(omx_muon_ns5_step)                  \
   X(omx_muon_ns5_step_batched) X(omx_muon_ns5_step_list) X(omx_muon_ns5_step_shapes) X(omx_adamw_step_batched) X(omx_accumulate_grads) X(omx_clip_grad_norm) X(omx_residual_add) X(omx_accumulate_grad) X(omx_scale_grad)        \
   X(omx_gelu_forward) X(omx_gelu_backward) X(omx_cached_attention_forward) X(omx_kv_cache_write) X(omx_token_windows)    \
-  X(omx_permute_0213) X(omx_silu_forward) X(omx_silu_backward) X(omx_mul_forward) X(omx_mul_backward)                    \
+  X(omx_permute_0213) X(omx_silu_forward) X(omx_silu_backward) X(omx_mul_forward) X(omx_mul_backward) X(omx_silu_mul_forward) X(omx_silu_mul_backward)                    \
   X(omx_rope_half_split_forward) X(omx_rope_half_split_backward) X(omx_rope_half_split_inplace)                          \
   X(omx_rope_half_split_pitched) X(omx_swiglu_forward) X(omx_swiglu_backward) X(omx_rms_qk_norm_forward)                 \
   X(omx_rms_qk_norm_backward) X(omx_per_head_sigmoid_gate_forward) X(omx_per_head_sigmoid_gate_backward)                 \

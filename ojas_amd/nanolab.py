@@ -158,9 +158,10 @@ class NanolabGraph:
             o = be.linear_forward(a["y"].reshape(N, H * D), self._blk(i, "mixer.o_proj.weight"))
             a["x1"], a["h2"] = add_norm(x, o, self._blk(i, "norm2.weight"))
             a["g_lin"] = be.linear_forward(a["h2"], self._blk(i, "ffn.gate.weight"))
-            a["g_act"] = be.silu_forward(a["g_lin"])
+            if not fused:
+                a["g_act"] = be.silu_forward(a["g_lin"])
             a["up"] = be.linear_forward(a["h2"], self._blk(i, "ffn.up.weight"))
-            a["m"] = be.mul_forward(a["g_act"], a["up"])
+            a["m"] = be.silu_mul_forward(a["g_lin"], a["up"]) if fused else be.mul_forward(a["g_act"], a["up"])
             down = be.linear_forward(a["m"], self._blk(i, "ffn.down.weight"))
             after = self._blk(i + 1, "norm1.weight") if i + 1 < s.n_layer else self.p["norm_f.weight"]
             x, h = add_norm(a["x1"], down, after)
@@ -180,9 +181,13 @@ class NanolabGraph:
         for i in reversed(range(s.n_layer)):
             a = acts[i]
             gm, grads[f"blocks.{i}.ffn.down.weight"] = be.linear_backward(a["m"], self._blk(i, "ffn.down.weight"), gx)
-            g_gact, g_up = be.mul_backward(a["g_act"], a["up"], gm)
+            if fused:
+                g_glin, g_up = be.silu_mul_backward(a["g_lin"], a["up"], gm)
+            else:
+                g_gact, g_up = be.mul_backward(a["g_act"], a["up"], gm)
             gh2, grads[f"blocks.{i}.ffn.up.weight"] = be.linear_backward(a["h2"], self._blk(i, "ffn.up.weight"), g_up)
-            g_glin = be.silu_backward(a["g_lin"], g_gact)
+            if not fused:
+                g_glin = be.silu_backward(a["g_lin"], g_gact)
             gh2, grads[f"blocks.{i}.ffn.gate.weight"] = linear_backward_onto(gh2, a["h2"], self._blk(i, "ffn.gate.weight"),
                                                                              g_glin)
             gx1, grads[f"blocks.{i}.norm2.weight"] = norm_backward_onto(gx, a["x1"], self._blk(i, "norm2.weight"), gh2)

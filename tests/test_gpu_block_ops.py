@@ -72,6 +72,29 @@ def test_silu_and_mul(be, n, bf16):
         assert np.array_equal(be.download(be.mul_forward(dx, db)), orc.mul_forward(x, b))
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 4096, 100004])
+def test_silu_mul_carries_the_bits_of_the_two_ops(be, n):
+    """One pass each way against the two ops; what is not finite is named as theirs."""
+    from ojas_amd.backend import OjasError
+
+    print(f"silu_mul n={n}", flush=True)
+    r = np.random.default_rng(n)
+    gate, up, gy = (be.upload((r.standard_normal(n) * 4).astype(np.float32)) for _ in range(3))
+    act = be.silu_forward(gate)
+    assert np.array_equal(be.download(be.silu_mul_forward(gate, up)), be.download(be.mul_forward(act, up)))
+    g_act, g_up = be.mul_backward(act, up, gy)
+    got = be.silu_mul_backward(gate, up, gy)
+    assert np.array_equal(be.download(got[0]), be.download(be.silu_backward(gate, g_act))) and np.array_equal(be.download(got[1]), be.download(g_up))
+    one = lambda v: be.upload(np.full(n, v, np.float32))
+    for call, name in ((lambda: be.silu_mul_forward(one(np.nan), one(1.0)), "silu_forward"), (lambda: be.silu_mul_forward(one(3e38), one(2.0)), "mul_forward"),
+                       (lambda: be.silu_mul_backward(one(1.0), one(3e38), one(3.0)), "mul_backward"),
+                       (lambda: be.silu_mul_backward(one(2.3), one(3.2e38), one(1.0)), "silu_backward")):
+        call()
+        with pytest.raises(OjasError) as e:
+            be.sync()
+        assert e.value.detail == name
+
+
 def test_silu_extremes_stay_finite(be):
     x = np.array([-200.0, -90.0, -20.0, -0.0, 0.0, 20.0, 90.0, 200.0], np.float32)
     y = be.download(be.silu_forward(be.upload(x)))
