@@ -243,8 +243,8 @@ class MiBackend(_native.Methods):
     def linear_backward_onto(self, g, x, w, gy):
         """g (f32, written to) + the input gradient of `linear_backward`, and its weight gradient."""
         rows, kin, nout = x.numel // x.shape[-1], x.shape[-1], w.shape[0]
-        if g.shape != x.shape or g.dtype != F32 or not (x.dtype == w.dtype == gy.dtype):
-            raise OjasError(DTYPE, "linear_backward_onto: an f32 sum of the input's shape, operands that share a dtype")
+        if not (x.dtype == w.dtype == gy.dtype):
+            raise OjasError(DTYPE, "linear_backward_onto: operands must share a dtype")
         gw = self.empty(w.shape, F32)
         _native.omx_linear_backward_onto(self._context, x, w, gy, x.dtype, g, gw, F32, rows, kin, nout)
         return g, gw
@@ -778,18 +778,12 @@ class MiBackend(_native.Methods):
 
     def silu_mul_forward(self, gate, up):
         """`mul_forward(silu_forward(gate), up)` in one pass (f32)."""
-        self._same("silu_mul_forward", gate, up)
-        if gate.dtype != F32:
-            raise OjasError(DTYPE, "silu_mul_forward: f32 operands")
         out = self.empty(gate.shape, F32)
         _native.omx_silu_mul_forward(self._context, gate, up, out, gate.numel)
         return out
 
     def silu_mul_backward(self, gate, up, gy):
         """Gradients of `silu_mul_forward` by gate and up."""
-        self._same("silu_mul_backward", gate, up, gy)
-        if gate.dtype != F32:
-            raise OjasError(DTYPE, "silu_mul_backward: f32 operands")
         g_gate, g_up = self.empty(gate.shape, F32), self.empty(gate.shape, F32)
         _native.omx_silu_mul_backward(self._context, gate, up, gy, g_gate, g_up, gate.numel)
         return g_gate, g_up
@@ -1049,6 +1043,7 @@ def _elementwise(op, n):
 _VALIDATED = {
     "linear_forward": (lambda x, w, *_a, **_k: shapes.linear_forward_dims(x, w), 2),
     "linear_backward": (lambda x, w, gy, *_a, **_k: shapes.linear_backward_dims(x, w, gy), 3),
+    "linear_backward_onto": (lambda g, x, w, gy: shapes.linear_backward_onto_dims(g, x, w, gy), 4),
     "causal_sdpa_forward": (lambda q, k, v, window=None, *_a, **_k: shapes.causal_sdpa_forward_dims(q, k, v, window), 3),
     "causal_sdpa_backward": (lambda q, k, v, out, lse, gy, window=None, *_a, **_k:
                              shapes.causal_sdpa_backward_dims(q, k, v, out, lse, gy, window), 6),
@@ -1080,6 +1075,8 @@ _VALIDATED = {
     "silu_backward": _elementwise("silu_backward", 2),
     "mul_forward": _elementwise("mul_forward", 2),
     "mul_backward": _elementwise("mul_backward", 3),
+    "silu_mul_forward": (lambda gate, up: shapes.silu_mul_dims("silu_mul_forward", gate, up), 2),
+    "silu_mul_backward": (lambda gate, up, gy: shapes.silu_mul_dims("silu_mul_backward", gate, up, gy), 3),
     "permute": (lambda x, axes: shapes.permute_dims(x, axes), 1),
     "per_head_sigmoid_gate_forward": (lambda x, w, b, a, *_a, **_k: shapes.per_head_sigmoid_gate_forward_dims(x, w, b, a), 4),
     "per_head_sigmoid_gate_forward_saving": (lambda x, w, b, a, *_a, **_k:

@@ -179,6 +179,19 @@ def linear_backward_dims(x, w, gy):
     return dims
 
 
+def linear_backward_onto_dims(g, x, w, gy):
+    """`linear_backward` into a sum: the sum (f32) first, its shape last."""
+    op = "linear_backward_onto"
+    _operand(op, g, (F32,))
+    for t in (x, w, gy):
+        _float(op, t)
+    dims = _linear(op, x, w)
+    if shape_of(gy) != dims[3]:
+        raise _refuse(op, f"grad shape {list(shape_of(gy))} != forward shape {list(dims[3])}")
+    _same(op, shape_of(x), shape_of(g))
+    return dims
+
+
 # ---- RMSNorm: shapes.rs:661-775 (the gradient's shape before eps and the layout)
 def _rms_layout(op, x, w, eps):
     if not math.isfinite(eps):
@@ -349,6 +362,13 @@ def value_residual_blend_backward_dims(v, v0, lam, gy):
 # ---- elementwise: shapes.rs:1348-1451, 1662-1690
 def elementwise_dims(op: str, *tensors) -> int:
     """silu / mul / residual_add / gelu / accumulate_grad: `same_shape` under the op's name."""
+    return _same_shape(op, tensors)
+
+
+def silu_mul_dims(op: str, *tensors) -> int:
+    """silu and mul in one pass: f32 only."""
+    for t in tensors:
+        _operand(op, t, (F32,))
     return _same_shape(op, tensors)
 
 

@@ -58,6 +58,13 @@ def cases():
     add("grad shape", "linear_backward", [f(3, 4), f(5, 4), f(3, 6)], (), 0, SHAPE)
     add("u32 grad", "linear_backward", [f(3, 4), f(5, 4), u(3, 5)], (), 0, DTYPE)
     add("weight rank 3", "linear_backward", [f(3, 4), f(5, 4, 1), f(3, 5)], (), 2, SHAPE)
+    onto = lambda g, x, w, gy: ("linear_backward_onto", [g, x, w, gy], ())
+    add("weight in-features under the input's", *onto(f(8, 64), f(8, 64), f(32, 16), f(8, 32)), 3, SHAPE)
+    add("fewer rows of gradient than of input", *onto(f(8, 64), f(8, 64), f(32, 64), f(4, 32)), 0, SHAPE)
+    add("gradient columns", *onto(f(3, 4), f(3, 4), f(5, 4), f(3, 6)), 0, SHAPE)
+    add("sum shape", *onto(f(3, 5), f(3, 4), f(5, 4), f(3, 5)), 1, SHAPE)
+    add("weight rank 3", *onto(f(3, 4), f(3, 4), f(5, 4, 1), f(3, 5)), 0, SHAPE)
+    add("u32 sum and grad shape: dtype of the sum first", *onto(u(3, 4), f(3, 4), f(5, 4), f(3, 6)), 1, DTYPE)
     # RMSNorm: the gradient's shape before eps and the layout (D8)
     add("weight length", "rms_norm_forward", [f(3, 8), f(7)], (1e-6,), 0, SHAPE)
     add("eps inf", "rms_norm_forward", [f(3, 8), f(8)], (float("inf"),), 0, NON_FINITE)
@@ -104,7 +111,8 @@ def cases():
     add("grad shape", "value_residual_blend_backward", [f(2, 3), f(2, 3), f(1), f(2, 4)], (), 0, SHAPE)
     # elementwise
     for op, n in (("silu_backward", 2), ("mul_forward", 2), ("mul_backward", 3), ("residual_add_forward", 2),
-                  ("gelu_erf_backward", 2), ("gelu_tanh_backward", 2), ("accumulate_grad", 2)):
+                  ("gelu_erf_backward", 2), ("gelu_tanh_backward", 2), ("accumulate_grad", 2), ("silu_mul_forward", 2),
+                  ("silu_mul_backward", 3)):
         add("shapes differ", op, [f(2, 3)] * (n - 1) + [f(3, 2)], (), 0, SHAPE)
         add("u32 operand", op, [f(2, 3)] * (n - 1) + [u(2, 3)], (), 0, DTYPE)
     for op in ("silu_forward", "gelu_erf_forward", "gelu_tanh_forward"):
