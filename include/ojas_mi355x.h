@@ -337,7 +337,9 @@ int32_t omx_rms_norm_backward_residual(omx_ctx* ctx, const void* x, int32_t x_dt
 /* From here on the weight gradients of rms_norm_backward and _residual and the bias gradients of
  * per_head_sigmoid_gate_backward and _deferred may wait, until omx_form_weight_sums forms them (`form` = 0: forgets them), as few
  * launches: each is a sum over some hundred partial rows, and a launch of its own takes 4 to 5 us whatever its size. Their
- * outputs are written by then, with the same bits; a non-finite one is reported under the op that it belongs to. `expected`: how many,
+ * outputs are written by then, with the same bits; a non-finite one is reported under the op that it belongs to. An op that reads one
+ * of them earlier finds what was there before. omx_sync and omx_download form what waits first, as do the omx_free of a block that one
+ * of them is in and another omx_defer_weight_sums. `expected`: how many,
  * for the size of the scratch (at most 64 MiB, given back to any allocation that would be refused once nothing waits); without
  * room they are formed at once. The reference's tape forms each where it stands (ojas-autograd/src/tape.rs:2565-2591). */
 int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected);

@@ -4,6 +4,8 @@
 // (upload/download, backend.rs:908-973), budget charging that refuses rather
 // than clamps (ojas-core/src/budget.rs:257-316), and the deferred non-finite
 // contract of a device backend (ojas-wgpu/src/backend.rs:35-73).
+#include <functional>
+
 #include "omx_common.h"
 
 static const char* kFaultNames[F_COUNT] = {
@@ -216,7 +218,7 @@ bool drop_extra(omx_ctx* ctx) {
   bool dropped = false;
   for (int slot : {kExtraSlot, kSumsSlot}) {
     void*& held = ctx->workspace[slot];
-    const bool in_use = slot == kExtraSlot ? ctx->extra_in_use : !ctx->sums.empty();
+    const bool in_use = slot == kExtraSlot ? ctx->extra_in_use : ctx->sums_used > 0;
     if (!held || in_use || ctx->workspace_captured[slot] || capturing(ctx)) continue;
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return dropped;
     ctx->budget_live -= ctx->allocations[held];
@@ -277,6 +279,16 @@ int32_t omx_free(omx_ctx* ctx, void* ptr) {
   auto it = ctx->allocations.find(ptr);
   if (it == ctx->allocations.end()) return omx_fail(ctx, OMX_PLACEMENT, "omx_free: pointer not from this context");
   const uint64_t bytes = it->second;
+  // A sum that waits would be written over whatever gets this block next.
+  const char* const from = static_cast<const char*>(ptr);
+  const std::less<const char*> before;
+  for (const OmxColumnSum& s : ctx->sums) {
+    const char* const at = reinterpret_cast<const char*>(s.out);
+    if (before(at, from) || !before(at, from + bytes)) continue;
+    const int32_t rc = omx_form_sums(ctx);
+    if (rc != OMX_OK) return rc;
+    break;
+  }
   ctx->budget_live -= bytes;
   ctx->allocations.erase(it);
   // Freeing for real would wait for the stream (work that still reads the buffer is on it) and for
@@ -346,6 +358,8 @@ namespace {
 // Waits for submitted work and reports a deferred fault; with the fault word come `n` (at most kReadback) bytes of `src`, to readback().
 // One launch and one wait: a copy of the fault word, a wait, a copy of the value and a wait were some 25 us between two halves of a step.
 int32_t sync_with(omx_ctx* ctx, const void* src, uint64_t n) {
+  const int32_t formed = omx_form_sums(ctx);
+  if (formed != OMX_OK) return formed;
   omx_launch(ctx, read_back_kernel, dim3(1), dim3(256), 0, ctx->fault, ctx->fault_host, static_cast<const char*>(src), readback(ctx), static_cast<int>(n));
   OMX_LAUNCH_CHECK(ctx, "read_back_kernel");
   const int32_t waited = wait(ctx);

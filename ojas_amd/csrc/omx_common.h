@@ -262,6 +262,8 @@ int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t 
                        float* scratch = nullptr, hipEvent_t stop = nullptr, bool wait = false);
 // Where sums wait and there is room, memory for their partial rows; else null.
 float* omx_partial_rows(omx_ctx* ctx, uint64_t blocks, uint64_t dim);
+// Forms every sum that waits.
+int32_t omx_form_sums(omx_ctx* ctx);
 // RMSNorm with 16-byte accesses for row widths 256..2048 (rmsvec.hip). `add` (forward) and
 // `add_in` / `gx16` (backward) are optional fused operands.
 bool omx_rms_vec_eligible(uint64_t dim, std::initializer_list<const void*> ptrs);

@@ -6,6 +6,8 @@
 //   rms_norm_*   ojas-cpu/src/norm.rs:24-204   (trait backend.rs:1658-1672)
 //   embedding_*  ojas-cpu/src/pointwise.rs:77-215 (trait backend.rs:1610-1626)
 //   argmax/topk  ojas-core/src/backend.rs:184-195,1514-1606
+#include <utility>
+
 #include "omx_common.h"
 
 namespace {
@@ -854,25 +856,23 @@ int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t 
   return OMX_OK;
 }
 
-namespace {
-// Forms every sum that waits, in the kernel's order of rows; its partial rows' memory is free again behind it.
-int32_t form_sums(omx_ctx* ctx) {
-  for (size_t first = 0; first < ctx->sums.size(); first += SUM_LIST) {
+// In the kernel's order of rows; the partial rows' memory is free again behind it. Nothing waits any more if a launch fails.
+int32_t omx_form_sums(omx_ctx* ctx) {
+  const std::vector<OmxColumnSum> sums = std::exchange(ctx->sums, {});
+  ctx->sums_used = 0;
+  for (size_t first = 0; first < sums.size(); first += SUM_LIST) {
     ColumnSumList list{};
-    const size_t count = std::min<size_t>(SUM_LIST, ctx->sums.size() - first);
+    const size_t count = std::min<size_t>(SUM_LIST, sums.size() - first);
     int dim = 0;
     for (size_t i = 0; i < count; ++i) {
-      list.of[i] = ctx->sums[first + i];
+      list.of[i] = sums[first + i];
       dim = std::max(dim, list.of[i].dim);
     }
     omx_launch(ctx, column_sum_list_kernel, dim3((dim + 63) / 64, static_cast<unsigned>(count)), dim3(1024), 0, list, ctx->fault);
     OMX_LAUNCH_CHECK(ctx, "column_sum_list_kernel");
   }
-  ctx->sums.clear();
-  ctx->sums_used = 0;
   return OMX_OK;
 }
-}  // namespace
 
 // The rows are those of the wide kernel, whose order the list keeps. Full memory is formed and used again. Rows of more than 1 MiB
 // are added at once: 16384 rows of 768 leave 1.5 MiB a norm, and the step that makes 25 of them, whose clock its products hold down,
@@ -882,7 +882,7 @@ float* omx_partial_rows(omx_ctx* ctx, uint64_t blocks, uint64_t dim) {
   constexpr uint64_t kMost = 64ull << 20;
   const uint64_t bytes = (blocks * dim * sizeof(float) + 255) / 256 * 256;
   if (bytes > 1ull << 20) return nullptr;
-  if (ctx->sums_used + bytes > ctx->workspace_bytes[kSumsSlot] && form_sums(ctx) != OMX_OK) return nullptr;
+  if (ctx->sums_used + bytes > ctx->workspace_bytes[kSumsSlot] && omx_form_sums(ctx) != OMX_OK) return nullptr;
   const uint64_t held = ctx->workspace_bytes[kSumsSlot];
   uint64_t want = held >= ctx->sums_used + bytes ? held : std::max(bytes, std::min(kMost, bytes * ctx->sums_expected));
   while (want >= 8 * bytes && !omx_workspace_fits(ctx, want, kSumsSlot)) want /= 2;
@@ -897,8 +897,8 @@ extern "C" {
 
 int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected) {
   OMX_REQUIRE_CTX(ctx);
-  ctx->sums.clear();
-  ctx->sums_used = 0;
+  const int32_t rc = omx_form_sums(ctx);
+  if (rc != OMX_OK) return rc;
   ctx->sums_expected = expected;
   ctx->sums_wait = true;
   return OMX_OK;
@@ -907,7 +907,7 @@ int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected) {
 int32_t omx_form_weight_sums(omx_ctx* ctx, int32_t form) {
   OMX_REQUIRE_CTX(ctx);
   ctx->sums_wait = false;
-  if (form) return form_sums(ctx);
+  if (form) return omx_form_sums(ctx);
   ctx->sums.clear();
   ctx->sums_used = 0;
   return OMX_OK;

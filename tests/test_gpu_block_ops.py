@@ -798,3 +798,42 @@ def test_weight_sums_that_wait_have_the_same_bits(count, budget_mib):
         assert np.array_equal(be.download(run()), want)  # formed at once again
     finally:
         be.close()
+
+
+def test_a_sum_that_waits_is_formed_before_anyone_could_miss_it():
+    """A download and a second `omx_defer_weight_sums` form what waits; so does the release of an output, whose block the next tensor
+    of its size gets; `omx_form_weight_sums(0)` forgets."""
+    from ojas_amd.backend import F32, MiBackend
+
+    print("sums that wait", flush=True)
+    rng = np.random.default_rng(0)
+    be = MiBackend(0)
+    try:
+        rows, dim = 2048, 512
+        x, gy = (be.upload(rng.standard_normal((rows, dim), dtype=np.float32)) for _ in range(2))
+        w, other = be.upload(rng.normal(1, 0.1, dim).astype(np.float32)), rng.standard_normal(dim, dtype=np.float32)
+        want = be.download(be.rms_norm_backward(x, w, gy, 1e-6)[1])
+
+        def wait():
+            be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(4)))
+            gx, gw = be.empty((rows, dim), F32), be.zeros((dim,))
+            be._check(be._lib.omx_rms_norm_backward(
+                be._ctx, be._p(x), C.c_int32(F32), be._p(w), be._p(gy), C.c_int32(F32), be._p(gx), C.c_int32(F32), be._p(gw),
+                C.c_uint64(rows), C.c_uint64(dim), C.c_float(1e-6)))
+            return gw
+
+        form = lambda how: be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(how)))
+        assert np.array_equal(be.download(wait()), want)
+        first = wait()
+        second = wait()
+        form(0)
+        assert np.array_equal(be.download(first), want) and not be.download(second).any()
+        gone = wait()
+        at = gone.ptr
+        del gone
+        here = [be.upload(other) for _ in range(8)]  # every parked block of this size
+        assert any(t.ptr == at for t in here)
+        form(1)
+        assert all(np.array_equal(be.download(t), other) for t in here)
+    finally:
+        be.close()
