@@ -12,6 +12,8 @@
 // One wave owns a row; lane l owns columns 256 j + 4 l .. + 3 of chunk j, so a
 // wave's loads are contiguous 1 KiB (f32) runs and the row stays in registers
 // between the sum-of-squares pass and the scaling pass.
+#include <utility>
+
 #include "omx_common.h"
 
 namespace {
@@ -462,7 +464,8 @@ int32_t omx_rms_norm_backward_residual(omx_ctx* ctx, const void* x, int32_t x_dt
     return omx_fail(ctx, OMX_DTYPE, "%s: dtype must be f32 or bf16", op);
   if (rows == 0 || dim == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
   if (!(eps == eps) || eps == INFINITY || eps == -INFINITY) return omx_fail(ctx, OMX_NON_FINITE, "%s", op);
-  if (!gw && !omx_rms_vec_eligible(dim, {x, w, gy, residual_grad, gx, gx_bf16})) {
+  const bool unasked = !gw && !omx_rms_vec_eligible(dim, {x, w, gy, residual_grad, gx, gx_bf16});
+  if (unasked) {
     // The separate kernels below always form the weight gradient: it goes to scratch.
     int32_t wrc = omx_workspace(ctx, dim * sizeof(float), &gw, 1);
     if (wrc != OMX_OK) return wrc;
@@ -471,8 +474,11 @@ int32_t omx_rms_norm_backward_residual(omx_ctx* ctx, const void* x, int32_t x_dt
     return omx_rms_backward_vec(ctx, x, x_dtype, static_cast<const float*>(w), gy, gy_dtype,
                                 static_cast<const float*>(residual_grad), gx, OMX_F32, gx_bf16,
                                 static_cast<float*>(gw), rows, dim, eps, omx_tag(ctx, F_RMS_BACKWARD));
-  // Other widths: the same three steps as separate kernels (gx is written, then added in place).
+  // Other widths: the same three steps as separate kernels (gx is written, then added in place). A sum into scratch, which another op
+  // may have by then, does not wait.
+  const bool sums_wait = std::exchange(ctx->sums_wait, ctx->sums_wait && !unasked);
   int32_t rc = omx_rms_norm_backward(ctx, x, x_dtype, w, gy, gy_dtype, gx, OMX_F32, gw, rows, dim, eps);
+  ctx->sums_wait = sums_wait;
   if (rc != OMX_OK) return rc;
   rc = omx_residual_add(ctx, residual_grad, OMX_F32, gx, OMX_F32, gx, OMX_F32, rows * dim);
   if (rc != OMX_OK) return rc;

@@ -837,3 +837,29 @@ def test_a_sum_that_waits_is_formed_before_anyone_could_miss_it():
         assert all(np.array_equal(be.download(t), other) for t in here)
     finally:
         be.close()
+
+
+def test_a_weight_sum_that_no_one_asked_for_does_not_wait():
+    """A residual whose rows are not on 16 bytes and no weight gradient: the separate kernels' goes to scratch, at once. With sums
+    waiting, the call takes the scratch of one without (a sum that waited would have rows of its own), and its gradient the same bits."""
+    from ojas_amd.backend import F32, MiBackend
+
+    print("weight sum into scratch", flush=True)
+    rng = np.random.default_rng(1)
+    be = MiBackend(0)
+    try:
+        rows, dim = 2048, 512
+        x, gy = (be.upload(rng.standard_normal((rows, dim), dtype=np.float32)) for _ in range(2))
+        w, res = be.upload(rng.normal(1, 0.1, dim).astype(np.float32)), be.upload(rng.standard_normal(rows * dim + 1, dtype=np.float32))
+        gx, live = [be.empty((rows, dim), F32) for _ in range(2)], []
+        for out in gx:
+            be._check(be._lib.omx_rms_norm_backward_residual(
+                be._ctx, be._p(x), C.c_int32(F32), be._p(w), be._p(gy), C.c_int32(F32), C.c_void_p(res.ptr + 4), be._p(out), None, None,
+                C.c_uint64(rows), C.c_uint64(dim), C.c_float(1e-6)))
+            live.append(be.budget()["live"])
+            be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(4)))
+        be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
+        assert live[0] == live[1]
+        assert np.array_equal(be.download(gx[0]), be.download(gx[1]))
+    finally:
+        be.close()
