@@ -340,7 +340,7 @@ int32_t omx_rms_norm_backward_residual(omx_ctx* ctx, const void* x, int32_t x_dt
  * outputs are written by then, with the same bits; a non-finite one is reported under the op that it belongs to. An op that reads one
  * of them earlier finds what was there before. omx_sync and omx_download form what waits first, as do the omx_free of a block that one
  * of them is in and another omx_defer_weight_sums. `expected`: how many,
- * for the size of the scratch (at most 64 MiB, given back to any allocation that would be refused once nothing waits); without
+ * for the size of the scratch (at most 64 MiB, given back to any allocation that would be refused, what waits formed); without
  * room they are formed at once. The reference's tape forms each where it stands (ojas-autograd/src/tape.rs:2565-2591). */
 int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected);
 int32_t omx_form_weight_sums(omx_ctx* ctx, int32_t form);

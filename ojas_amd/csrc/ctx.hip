@@ -212,14 +212,19 @@ bool capturing(const omx_ctx* ctx) {
   return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 
-// Gives workspaces kExtraSlot and kSumsSlot back, unless the op that runs or sums that wait use them or a graph holds their
-// address. Whether there was one.
+// Whether drop_extra gives workspace `slot` (kExtraSlot or kSumsSlot) back: not while the op that runs uses it, a graph holds its
+// address or a capture is on.
+bool droppable(const omx_ctx* ctx, int slot) {
+  return ctx->workspace[slot] && !(slot == kExtraSlot && ctx->extra_in_use) && !ctx->workspace_captured[slot] && !capturing(ctx);
+}
+
+// Gives workspaces kExtraSlot and kSumsSlot back, with the sums that wait there formed. Whether there was one. (No op allocates
+// between omx_partial_rows and its omx_column_sum.)
 bool drop_extra(omx_ctx* ctx) {
   bool dropped = false;
   for (int slot : {kExtraSlot, kSumsSlot}) {
     void*& held = ctx->workspace[slot];
-    const bool in_use = slot == kExtraSlot ? ctx->extra_in_use : ctx->sums_used > 0;
-    if (!held || in_use || ctx->workspace_captured[slot] || capturing(ctx)) continue;
+    if (!droppable(ctx, slot) || (slot == kSumsSlot && omx_form_sums(ctx) != OMX_OK)) continue;
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return dropped;
     ctx->budget_live -= ctx->allocations[held];
     ctx->allocations.erase(held);

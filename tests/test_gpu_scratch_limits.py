@@ -259,3 +259,29 @@ def test_a_widened_weight_makes_room_for_what_is_allocated_next():
         del rest
     finally:
         be.close()
+
+
+def test_sums_that_wait_make_room_for_what_is_allocated_next():
+    """The partial rows of a norm's weight gradient are scratch: an allocation that needs their room gets it, and the gradient is formed."""
+    from ojas_amd.backend import F32, MiBackend
+
+    print("an allocation while sums wait", flush=True)
+    r = np.random.default_rng(5)
+    be = MiBackend(0, budget_bytes=32 << 20)
+    try:
+        rows, dim = 2048, 512
+        x, gy = (be.upload(r.standard_normal((rows, dim), dtype=np.float32)) for _ in range(2))
+        w, gx, gw = be.upload(r.normal(1, 0.1, dim).astype(np.float32)), be.empty((rows, dim), F32), be.zeros((dim,))
+        want = be.download(be.rms_norm_backward(x, w, gy, 1e-6)[1])
+        held = be.budget()["live"]
+        be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(64)))
+        be._check(be._lib.omx_rms_norm_backward(
+            be._ctx, be._p(x), C.c_int32(F32), be._p(w), be._p(gy), C.c_int32(F32), be._p(gx), C.c_int32(F32), be._p(gw), C.c_uint64(rows),
+            C.c_uint64(dim), C.c_float(1e-6)))
+        assert be.budget()["live"] - held >= 1 << 20
+        rest = be.empty((((32 << 20) - be.budget()["live"] + (1 << 20)) // 4,), F32)  # a MiB more than there is
+        be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
+        assert np.array_equal(be.download(gw), want)
+        del rest
+    finally:
+        be.close()
