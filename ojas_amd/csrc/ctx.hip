@@ -430,7 +430,11 @@ uint64_t workspace_size(uint64_t bytes) { return (bytes + (1ull << 20) - 1) & ~(
 bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot) {
   const uint64_t held = ctx->workspace_bytes[slot];
   if (bytes <= held || ctx->budget_limit == 0) return true;
-  const uint64_t back = ctx->workspace_captured[slot] || capturing(ctx) ? 0 : held;  // what growing it gives back
+  uint64_t back = ctx->workspace_captured[slot] || capturing(ctx) ? 0 : held;  // what growing it gives back
+  // An op's plan does not depend on what others can do without: omx_alloc takes that back for it.
+  if (slot != kExtraSlot && slot != kSumsSlot)
+    for (int extra : {kExtraSlot, kSumsSlot})
+      if (droppable(ctx, extra)) back += ctx->workspace_bytes[extra];
   return ctx->budget_live - back + workspace_size(bytes) <= ctx->budget_limit;
 }
 

@@ -206,7 +206,8 @@ int32_t omx_hip_fail(omx_ctx* ctx, hipError_t err, const char* what);
 constexpr int kExtraSlot = 3, kSumsSlot = 4;
 // Grows workspace `slot` to at least `bytes` (budget-charged).
 int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot = 0);
-// Whether the budget has room for workspace `slot` at that size (for an op that can do with less).
+// Whether the budget has room for workspace `slot` at that size (for an op that can do with less), counting what kExtraSlot and kSumsSlot
+// would give back.
 bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot = 0);
 // Workspace `slot` for an op that can do without: null where the budget or the device lacks the room, and where a capture would have to
 // allocate it.

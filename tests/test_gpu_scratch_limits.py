@@ -261,6 +261,36 @@ def test_a_widened_weight_makes_room_for_what_is_allocated_next():
         be.close()
 
 
+def test_a_plan_does_not_depend_on_scratch_that_can_be_given_back():
+    """A Muon list takes as many matrices at a time as the budget has room for, and as many after an int8 product has left its widened
+    weight behind: the same scratch in the end, the same bits."""
+    from ojas_amd.backend import BF16, MiBackend, MuonNs5Config
+
+    print("muon list beside a widened weight", flush=True)
+    r = np.random.default_rng(4)
+    n, d = 8, (256, 512)
+    ps, gs, ms = ([(r.standard_normal(d) * s).astype(np.float32) for _ in range(n)] for s in (0.1, 0.05, 0.01))
+    x, codes = r.normal(0, 1, (64, 1024)).astype(np.float32), r.integers(-127, 128, (2048, 1024)).astype(np.int8)
+    scales = r.uniform(1e-4, 1e-3, (2048, 32)).astype(np.float32)
+    out = []
+    for widened in (False, True):
+        be = MiBackend(0, budget_bytes=3 * n * 4 * d[0] * d[1] + (14 << 20))  # five matrices' scratch
+        try:
+            if widened:
+                be.set_option("q8_widen", 1)
+                before = be.budget()["live"]
+                be.linear_i8_group_forward(be.upload(x, BF16), be.upload(codes), be.upload(scales))
+                be.sync()
+                assert be.budget()["live"] - before == 4 << 20
+            dp, dg, dm = ([be.upload(a) for a in xs] for xs in (ps, gs, ms))
+            be.muon_ns5_step_list(dp, dg, dm, MuonNs5Config(0.02, 0.95, 0.1, 1, 0))
+            out.append((be.budget()["live"], [be.download(t) for t in dp + dm]))
+        finally:
+            be.close()
+    assert out[0][0] == out[1][0]
+    assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
+
+
 def test_sums_that_wait_make_room_for_what_is_allocated_next():
     """The partial rows of a norm's weight gradient are scratch: an allocation that needs their room gets it, and the gradient is formed."""
     from ojas_amd.backend import F32, MiBackend
