@@ -160,7 +160,9 @@ int32_t omx_gemm_pitched_strided_batch(omx_ctx* ctx, const void* a, uint64_t a_r
  * per-channel form of ojas-cpu/src/quant_sparse.rs:284-346 applied to groups; group must be 32).
  * The codes are widened inside the product, on their way from HBM to the matrix units, or, where that is
  * ahead and the budget has room, into scratch that the next product writes over (at most 1 GiB, given back to any
- * allocation that would be refused; the same bits either way). No bf16 copy of a weight is kept. In the reference a quantised base reaches the graph as
+ * allocation that would be refused). Either way the same weight, and f32 sums; over the copy a product of few rows, few columns or few
+ * tiles over a long reduction may add them in another order, so its last bits can depend on whether there was room. No bf16 copy of a
+ * weight is kept. In the reference a quantised base reaches the graph as
  * dequantise -> linear_forward (ojas-autograd/src/tape.rs:1514-1518, backend.rs:2586); these two
  * entry points serve that pair of calls for a frozen base, forward and input gradient (a frozen
  * weight has no gradient, ojas-model/src/lora.rs:4-8).

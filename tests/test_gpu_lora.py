@@ -78,7 +78,8 @@ def test_linear_i8_group_backward_input(be, rows, kin, nout, with_add):
     (33, 128, 64, 16, 0, True), (257, 128, 384, 16, 128, True), (1025, 512, 768, 32, 256, True), (300, 192, 320, 16, 0, False),
     (4100, 256, 512, 0, 0, True), (8193, 768, 2304, 16, 768, True)])
 def test_linear_i8_group_over_a_widened_copy(be, rows, kin, nout, rank, block, blocked, backward):
-    # A weight widened in scratch gives the bits of one widened on its way: the same bf16 values, the same order of sums.
+    # A weight widened in scratch gives the bits of one widened on its way where K is not shared: the same bf16 values, the same order
+    # of sums.
     from ojas_amd.backend import BF16, F32
 
     print(f"q8 widened rows={rows} kin={kin} nout={nout} rank={rank} backward={backward}", flush=True)
@@ -105,6 +106,43 @@ def test_linear_i8_group_over_a_widened_copy(be, rows, kin, nout, rank, block, b
     finally:
         be.set_option("q8_widen", -1)
     assert np.array_equal(got[0], got[1])
+
+
+# Few tiles over a long reduction, few rows and few columns: over the copy K is shared between launches or between waves.
+@pytest.mark.parametrize("backward", [False, True])
+@pytest.mark.parametrize("rows,kin,nout,rank", [(256, 8192, 2048, 16), (300, 4096, 1024, 32), (64, 2048, 6144, 0), (17, 4096, 256, 0),
+                                                (1500, 2048, 64, 0), (1100, 128, 2048, 0)])
+def test_linear_i8_group_over_a_widened_copy_that_shares_k(be, rows, kin, nout, rank, backward):
+    """Both ways against the f64 product of the same bf16 operands: k exact products and as many f32 additions, (k + rank) 2^-23
+    sum |a||b| with room for an accumulator that cuts off, an input gradient's store to bf16 on top; and the copy's error no larger."""
+    from ojas_amd.backend import BF16, F32
+
+    print(f"q8 widened, K shared: rows={rows} kin={kin} nout={nout} rank={rank} backward={backward}", flush=True)
+    rng = np.random.default_rng(rows + nout)
+    codes, scales = rng.integers(-127, 128, (nout, kin)).astype(np.int8), rng.uniform(1e-4, 1e-3, (nout, kin // 32)).astype(np.float32)
+    w = orc.round_bf16(codes * np.repeat(scales, 32, 1)).astype(np.float64)
+    w = w if backward else w.T
+    x = orc.round_bf16(rng.normal(0, 1, (rows, len(w))).astype(np.float32))
+    dx, low_rank = be.upload(x, BF16), None
+    want, size = x.astype(np.float64) @ w, np.abs(x).astype(np.float64) @ np.abs(w)
+    if rank:
+        h, up = (orc.round_bf16(rng.normal(0, s, (n, rank)).astype(np.float32)) for s, n in ((1, rows), (0.1, w.shape[1])))
+        low_rank = (be.upload(h, BF16), be.upload(up, BF16), 0)
+        want, size = want + h.astype(np.float64) @ up.T, size + np.abs(h).astype(np.float64) @ np.abs(up.T)
+    bound = (len(w) + rank) * 2.0 ** -23 * size
+    dc, ds = be.pack_i8_group(be.upload(codes), be.upload(scales))
+    errors = []
+    try:
+        for widen in (0, 1):
+            be.set_option("q8_widen", widen)
+            y = (be.linear_i8_group_backward_input(dc, ds, dx, blocked=True, low_rank=low_rank) if backward else
+                 be.linear_i8_group_forward(dx, dc, ds, blocked=True, low_rank=low_rank, out_dtype=F32))
+            off = np.abs(be.download_f32(y) - want)
+            assert (off <= bound + (2.0 ** -8 * (np.abs(want) + bound) if backward else 0)).all()
+            errors.append(np.linalg.norm(off))
+    finally:
+        be.set_option("q8_widen", -1)
+    assert errors[1] <= 1.01 * errors[0], errors
 
 
 def test_linear_i8_group_scale_per_group_is_exact(be):
