@@ -290,13 +290,15 @@ MIXES = [
     [(64, 48, 2), (36, 100, 1), (100, 36, 1), (130, 70, 2), (4, 4, 1), (4, 32, 1), (32, 4, 1), (12, 20, 1), (8, 72, 1), (60, 60, 1), (68, 44, 1)],
     [(32, 32, 50), (32, 64, 30)],
 ]
-# f32: third products on 64 x 64 tiles that end inside one, over one step of K and over three, beside some on 32 x 32. (The bf16
+# f32: third products of many shapes and tiles that are too short for 64 x 64 ones (LARGE_TILES), and on 64 x 64 tiles that end inside
+# one, over six, seven and eight steps of K, beside some on 32 x 32 (LONG_TILES). (The bf16
 # iteration has launches of its own for each shape. Its gate is not meant for these: a 96 x 100 matrix of random values has singular
 # values from some 0.01 of its largest, which five iterations raise by up to 3.4 each with every operand rounded to 2^-9.)
 LARGE_TILES = [(96, 100, 16), (100, 96, 12), (224, 32, 8), (32, 224, 2), (4, 100, 2), (60, 52, 3)]
+LONG_TILES = [(192, 200, 10), (200, 192, 5), (224, 292, 2), (292, 256, 2), (160, 200, 3), (4, 100, 2)]
 
 
-@pytest.mark.parametrize("mix,bf16", [(mix, bf16) for bf16 in (0, 1) for mix in MIXES] + [(LARGE_TILES, 0)])
+@pytest.mark.parametrize("mix,bf16", [(mix, bf16) for bf16 in (0, 1) for mix in MIXES] + [(LARGE_TILES, 0), (LONG_TILES, 0)])
 def test_shapes_step_matches_the_oracle_per_tensor(be, mix, bf16):
     """`muon_ns5_step_shapes` at the single op's gates (momentum bit for bit; update 2e-3 of its largest element in f32,
     5e-2 with the bf16 iteration), tensors of one shape apart from each other in the call."""
@@ -380,3 +382,21 @@ def test_shapes_step_takes_the_scratch_there_is():
         upd_gpu, upd_cpu = small.download(dp[i]) - ps[i] * decay, op - ps[i] * decay
         assert np.max(np.abs(upd_gpu - upd_cpu)) <= 2e-3 * np.max(np.abs(upd_cpu)), i
     small.close()
+
+
+@pytest.mark.parametrize("dim,same", [(128, True), (160, True), (192, False)])
+def test_products_below_192_keep_their_tiles_whatever_the_count(be, dim, same):
+    """64 x 64 tiles, whose sums over a short K are less exact than those of 32 x 32 ones, are for K >= 192: below, a matrix steps to
+    the same bits among forty of its shape as among two."""
+    from ojas_amd.backend import MuonNs5Config
+
+    print(f"muon shapes {dim}", flush=True)
+    r = np.random.default_rng(dim)
+    cfg, got = MuonNs5Config(0.02, 0.95, 0.1, 1, 0), []
+    many = [(dim, dim)] * 40 + [(32, 36)]
+    ps, gs, ms = ([(r.standard_normal(d) * s).astype(np.float32) for d in many] for s in (0.1, 0.05, 0.01))
+    for part in (slice(0, 41), slice(39, 41)):
+        dp, dg, dm = ([be.upload(x) for x in xs[part]] for xs in (ps, gs, ms))
+        be.muon_ns5_step_shapes(dp, dg, dm, cfg)
+        got.append(be.download(dp[-2]))
+    assert np.array_equal(*got) == same
