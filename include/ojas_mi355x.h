@@ -728,7 +728,9 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value);
  * begin timestamp of its first kernel, the end timestamp of its last: the
  * MFMA kernel, or the split-K reduce after it), on the context's stream. The
  * report waits for the stream, sums the products' durations and their
- * 2*M*N*K FLOPs, and clears the record. */
+ * 2*M*N*K FLOPs, and clears the record. Products that go out in one launch
+ * (both gradients of a linear layer, the Newton-Schulz products of several
+ * shapes) count as one. */
 int32_t omx_profile_gemm(omx_ctx* ctx, int32_t enable);
 int32_t omx_profile_gemm_report(omx_ctx* ctx, uint64_t* launches, double* total_ms,
                                 double* total_flops);

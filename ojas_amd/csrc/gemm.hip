@@ -513,7 +513,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 bool omx_linear_backward_pair(omx_ctx* ctx, const float* x, const float* w, const float* gy, float* gx, float* gw, uint64_t rows, uint64_t in,
                               uint64_t out, bool onto, int32_t* rc) {
   const uint64_t most = 0x7fffffff;
-  if (ctx->gemm_f32_pair == 0 || ctx->gemm_dma_mode != 1 || ctx->gemm_f32_tile >= 0 || ctx->profile_gemm || rows > most || in > most || out > most)
+  if (ctx->gemm_f32_pair == 0 || ctx->gemm_dma_mode != 1 || ctx->gemm_f32_tile >= 0 || rows > most || in > most || out > most)
     return false;
   // (One after the other, the second product reads what the first one stored.)
   auto apart = [](const float* a, uint64_t an, const float* b, uint64_t bn) {
@@ -566,7 +566,11 @@ bool omx_linear_backward_pair(omx_ctx* ctx, const float* x, const float* w, cons
   gemm_w.tag = gemm_w.act_tag = omx_tag(ctx, F_LINEAR_BACKWARD);
   gemm_x.accumulate = onto;
   gemm_x.tag = gemm_x.act_tag = onto ? omx_tag(ctx, F_GEMM) : gemm_w.tag;  // (named as the two calls it stands for)
+  omx_ctx::TimedLaunch timed{};
+  *rc = omx_timing_begin(ctx, 4.0 * static_cast<double>(rows) * static_cast<double>(in) * static_cast<double>(out), &timed);
+  if (*rc != OMX_OK) return true;
   *rc = ctx->gemm_f32_pair < 0 && dma32 >= 0 ? omx_gemm_dma32_pair(ctx, gemm_x, gemm_w, dma32) : omx_gemm_frag32_pair(ctx, gemm_x, gemm_w, tile);
+  omx_timing_end(ctx, *rc == OMX_OK, timed);
   return true;
 }
 

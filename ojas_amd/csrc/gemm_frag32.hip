@@ -423,16 +423,11 @@ int32_t launch_pair(omx_ctx* ctx, GemmArgs x, GemmArgs w) {
   w.tiles_m = (w.M + 16 * WM - 1) / (16 * WM);
   w.tiles_n = (w.N + 16 * WN - 1) / (16 * WN);
   const int x_first = (w.tiles_m * w.tiles_n + 7) & ~7;
-  omx_launch(ctx, kernel, dim3(static_cast<unsigned>(x_first + x.tiles_m * x.tiles_n)), dim3(PAIR_WAVES * 64), smem, x, w, x_first);
+  omx_launch_timed(ctx, kernel, dim3(static_cast<unsigned>(x_first + x.tiles_m * x.tiles_n)), dim3(PAIR_WAVES * 64), smem, ctx->timing_start,
+                   ctx->timing_stop, x, w, x_first);
   OMX_LAUNCH_CHECK(ctx, "gemm_frag32_pair_kernel");
   return OMX_OK;
 }
-}  // namespace
-
-// us: a fixed part, then what the tiles take side by side over the compute units and the longest walk of one, squares added. Fitted
-// over 326 layers of 24 .. 6000 rows and 12 .. 1600 columns, each on all four pairs (rms 7 %); the tiles it chooses are 1.4 % behind
-// the best of the four on average (32 x 32 for both 17 %).
-namespace {
 template <int KG>
 int32_t launch_dma_pair(omx_ctx* ctx, GemmArgs x, GemmArgs w) {
   using D = PairDma<KG>;
@@ -444,10 +439,14 @@ int32_t launch_dma_pair(omx_ctx* ctx, GemmArgs x, GemmArgs w) {
   w.tiles_m = (w.M + 31) / 32;
   w.tiles_n = (w.N + 31) / 32;
   const int x_first = (w.tiles_m * w.tiles_n + 7) & ~7;
-  omx_launch(ctx, (gemm_dma32_pair_kernel<KG>), dim3(static_cast<unsigned>(x_first + x.tiles_m * x.tiles_n)), dim3(PAIR_WAVES * 64), smem, x, w, x_first);
+  omx_launch_timed(ctx, gemm_dma32_pair_kernel<KG>, dim3(static_cast<unsigned>(x_first + x.tiles_m * x.tiles_n)), dim3(PAIR_WAVES * 64), smem,
+                   ctx->timing_start, ctx->timing_stop, x, w, x_first);
   OMX_LAUNCH_CHECK(ctx, "gemm_dma32_pair_kernel");
   return OMX_OK;
 }
+// us: a fixed part, then what the tiles take side by side over the compute units and the longest walk of one, squares added. Fitted
+// over 326 layers of 24 .. 6000 rows and 12 .. 1600 columns, each on all four pairs (rms 7 %); the tiles it chooses are 1.4 % behind
+// the best of the four on average (32 x 32 for both 17 %).
 constexpr double PAIR_US = 2.83;
 struct PairTile {
   int xm, xn, wm, wn;
@@ -520,9 +519,13 @@ int32_t omx_gemm_frag32_group(omx_ctx* ctx, const OmxGemmProduct* products, int 
   q.fault = ctx->fault;
   q.tag = tag;
   uint64_t large_tiles = 0;
-  for (int i = 0; i < count && !symmetric; ++i)
-    if (group_fits_dma(products[i]))
-      large_tiles += ((products[i].m + GROUP_DMA_TILE - 1) / GROUP_DMA_TILE) * ((products[i].n + GROUP_DMA_TILE - 1) / GROUP_DMA_TILE) * products[i].batches;
+  double flops = 0.0;
+  for (int i = 0; i < count; ++i) {
+    const OmxGemmProduct& p = products[i];
+    flops += 2.0 * static_cast<double>(p.m) * static_cast<double>(p.n) * static_cast<double>(p.k) * static_cast<double>(p.batches);
+    if (!symmetric && group_fits_dma(p))
+      large_tiles += ((p.m + GROUP_DMA_TILE - 1) / GROUP_DMA_TILE) * ((p.n + GROUP_DMA_TILE - 1) / GROUP_DMA_TILE) * p.batches;
+  }
   const bool large = 2 * large_tiles >= static_cast<uint64_t>(ctx->cu_count > 0 ? ctx->cu_count : 256);
   int at = 0;
   for (int i = 0; i < count; ++i) {
@@ -549,7 +552,14 @@ int32_t omx_gemm_frag32_group(omx_ctx* ctx, const OmxGemmProduct* products, int 
     q.first[i] = 0x7fffffff;
     q.product[i] = FragProduct{};
   }
-  omx_launch(ctx, gemm_frag32_group_kernel, dim3(static_cast<unsigned>(at)), dim3(GROUP_WAVES * 64), 0, q);
-  OMX_LAUNCH_CHECK(ctx, "gemm_frag32_group_kernel");
-  return OMX_OK;
+  omx_ctx::TimedLaunch timed{};
+  int32_t rc = omx_timing_begin(ctx, flops, &timed);
+  if (rc != OMX_OK) return rc;
+  rc = [&]() -> int32_t {
+    omx_launch_timed(ctx, gemm_frag32_group_kernel, dim3(static_cast<unsigned>(at)), dim3(GROUP_WAVES * 64), 0, ctx->timing_start, ctx->timing_stop, q);
+    OMX_LAUNCH_CHECK(ctx, "gemm_frag32_group_kernel");
+    return OMX_OK;
+  }();
+  omx_timing_end(ctx, rc == OMX_OK, timed);
+  return rc;
 }

@@ -748,3 +748,35 @@ def test_both_gradients_in_one_launch(be, pair, rows, kin, nout):
         assert e.value.detail == "linear_backward"
     finally:
         be.set_option("gemm_f32_pair", -1)
+
+
+def test_products_of_one_launch_are_in_the_profile(be):
+    """Both gradients of a linear layer and the Newton-Schulz products of two shapes: one entry a launch with the products' operations,
+    and the bits of a call that is not timed."""
+    from ojas_amd.backend import MuonNs5Config
+
+    print("profile of products together", flush=True)
+    be.set_option("gemm_dma", 1)
+    r = np.random.default_rng(3)
+    x, w, gy = (be.upload(r.standard_normal(s, dtype=np.float32)) for s in ((1024, 256), (128, 256), (1024, 128)))
+    dims = [(64, 48), (36, 100), (64, 48)]
+    host = [[(r.standard_normal(d) * s).astype(np.float32) for d in dims] for s in (0.1, 0.05, 0.01)]
+
+    def step():
+        out = list(be.linear_backward(x, w, gy))
+        p, g, m = ([be.upload(a) for a in xs] for xs in host)
+        be.muon_ns5_step_shapes(p, g, m, MuonNs5Config(0.02, 0.95, 0.1, 1, 0))
+        return [be.download(t) for t in out + p]
+
+    want = step()
+    try:
+        be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(1)))
+        got = step()
+        launches, ms, flops = C.c_uint64(), C.c_double(), C.c_double()
+        be._check(be._lib.omx_profile_gemm_report(be._ctx, C.byref(launches), C.byref(ms), C.byref(flops)))
+    finally:
+        be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(0)))
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    assert launches.value == 1 + 15 and ms.value > 0
+    ns = sum(5 * 2.0 * (2 * min(d) ** 2 * max(d) + min(d) ** 3) for d in dims)
+    assert flops.value == 4.0 * 1024 * 256 * 128 + ns
