@@ -469,7 +469,7 @@ int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void
 // 1689 / 1601 (1629).
 constexpr uint64_t MU_TOGETHER = 1ull << 30;
 bool goes_together(omx_ctx* ctx, uint64_t rows, uint64_t cols, uint64_t count, bool bf16) {
-  if (bf16 || !ctx->muon_fused_sums || rows % 4 != 0 || cols % 4 != 0 || rows > 1u << 15 || cols > 1u << 15) return false;
+  if (bf16 || !ctx->muon_fused_sums || ctx->gemm_dma_mode != 1 || ctx->gemm_f32_tile >= 0 /* a forced kernel or tile */ || rows % 4 != 0 || cols % 4 != 0 || rows > 1u << 15 || cols > 1u << 15) return false;
   return std::min(rows, cols) * rows * cols <= MU_TOGETHER / count;
 }
 

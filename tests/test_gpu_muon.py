@@ -7,6 +7,8 @@ re-ordered f32 sums, gated like the reference's device runs (1e-4 of the
 largest value, ojas-wgpu/tests/common/mod.rs:11); the bf16 iteration is gated
 at the reference's own bf16-NS5 parameter bound (5e-2 of the update's scale,
 ojas-oracle/src/parity.rs:29-74)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -400,3 +402,31 @@ def test_products_below_192_keep_their_tiles_whatever_the_count(be, dim, same):
         be.muon_ns5_step_shapes(dp, dg, dm, cfg)
         got.append(be.download(dp[-2]))
     assert np.array_equal(*got) == same
+
+
+@pytest.mark.parametrize("option,value", [("gemm_f32", 2), ("gemm_dma", 0)])
+def test_a_forced_kernel_takes_the_products_of_several_shapes_too(be, option, value):
+    """Under an option that forces a tile or the register-staged kernel, each shape's products go out as they do in a list of its own."""
+    from ojas_amd.backend import MuonNs5Config
+
+    print(f"muon shapes {option}={value}", flush=True)
+    r = np.random.default_rng(value)
+    dims = [(64, 48), (36, 100), (64, 48)]
+    ps, gs, ms = ([(r.standard_normal(d) * s).astype(np.float32) for d in dims] for s in (0.1, 0.05, 0.01))
+    cfg = MuonNs5Config(0.02, 0.95, 0.1, 1, 0)
+    launches = C.c_uint64()
+    be.set_option(option, value)
+    try:
+        be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(1)))
+        got = [[be.upload(x) for x in xs] for xs in (ps, gs, ms)]
+        be.muon_ns5_step_shapes(*got, cfg)
+        be._check(be._lib.omx_profile_gemm_report(be._ctx, C.byref(launches), None, None))
+        be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(0)))
+        for shape in ((0, 2), (1,)):
+            want = [[be.upload(xs[i]) for i in shape] for xs in (ps, gs, ms)]
+            be.muon_ns5_step_list(*want, cfg)
+            assert all(np.array_equal(be.download(got[0][i]), be.download(p)) for i, p in zip(shape, want[0]))
+    finally:
+        be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(0)))
+        be.set_option(option, -1 if option == "gemm_f32" else 1)
+    assert launches.value == 2 * 15
