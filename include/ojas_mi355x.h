@@ -113,7 +113,8 @@ int32_t omx_linear_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const v
                            int32_t w_dtype, void* y, int32_t y_dtype, uint64_t rows,
                            uint64_t in_features, uint64_t out_features);
 /* BackendModule::linear_backward (backend.rs:1631): gx = gy.W, gw = gy^T.x.
- * gx or gw may be NULL (linear_backward_input, backend.rs:1643-1656). */
+ * gx or gw may be NULL (linear_backward_input, backend.rs:1643-1656). gx has the bits of a call for it alone; gw, where both are asked
+ * for in f32, may have its sums in another order than a call for it alone (at least as close to the exact ones). */
 int32_t omx_linear_backward(omx_ctx* ctx, const void* x, const void* w, const void* gy,
                             int32_t operand_dtype, void* gx, int32_t gx_dtype, void* gw,
                             int32_t gw_dtype, uint64_t rows, uint64_t in_features,

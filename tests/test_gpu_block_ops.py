@@ -792,9 +792,12 @@ def test_weight_sums_that_wait_have_the_same_bits(count, budget_mib):
 
         want = be.download(run())
         be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(count)))
-        waiting = run()
+        waiting, before = run(), be.empty((count, 512), F32)
+        be._check(be._lib.omx_copy(be._ctx, be._p(before), be._p(waiting), C.c_uint64(before.nbytes)))
         be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
         assert np.array_equal(be.download(waiting), want)
+        if not budget_mib:  # none of three had been formed, nor the last of 70 (whose rows fill the memory that the first one's size gave)
+            assert not be.download(before)[0 if count == 3 else -1:].any()
         assert np.array_equal(be.download(run()), want)  # formed at once again
     finally:
         be.close()
@@ -861,5 +864,43 @@ def test_a_weight_sum_that_no_one_asked_for_does_not_wait():
         be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
         assert live[0] == live[1]
         assert np.array_equal(be.download(gx[0]), be.download(gx[1]))
+    finally:
+        be.close()
+
+
+def test_gate_bias_sums_wait_and_overflows_are_named():
+    """The gate's bias gradient waits as the norms' do; a sum of finite rows that is not finite is reported under its own op."""
+    from ojas_amd.backend import F32, MiBackend, OjasError
+
+    print("gate bias sums that wait", flush=True)
+    rng = np.random.default_rng(2)
+    be = MiBackend(0)
+    try:
+        x, w, b = (be.upload(0.3 * rng.standard_normal(s, dtype=np.float32)) for s in ((1, 900, 32), (4, 32), (4,)))
+        attn, gy = (be.upload(rng.standard_normal((1, 900, 4, 16), dtype=np.float32)) for _ in range(2))
+        defer = lambda: be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(2)))
+        form = lambda: be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
+        want = [be.download(t) for t in be.per_head_sigmoid_gate_backward(x, w, b, attn, gy)]
+        parked = [be.zeros((4,)) for _ in range(8)]  # (the next tensors of this size get these blocks)
+        before = be.upload(np.ones(4, np.float32))
+        del parked
+        defer()
+        got = be.per_head_sigmoid_gate_backward(x, w, b, attn, gy)
+        be._check(be._lib.omx_copy(be._ctx, be._p(before), be._p(got[2]), C.c_uint64(16)))
+        form()
+        assert all(np.array_equal(be.download(a), c) for a, c in zip(got, want))
+        assert not be.download(before).any()
+        rows, dim = 2048, 512
+        ones, steep = np.ones((rows, dim), np.float32), np.zeros((rows, dim), np.float32)
+        steep[:, 7] = 1e36  # 2e39 in all, 6e37 in a block's rows
+        dx, dg, dw, gx, gw = be.upload(ones), be.upload(steep), be.upload(ones[0]), be.empty((rows, dim), F32), be.empty((dim,), F32)
+        defer()
+        be._check(be._lib.omx_rms_norm_backward(be._ctx, be._p(dx), C.c_int32(F32), be._p(dw), be._p(dg), C.c_int32(F32), be._p(gx), C.c_int32(F32),
+                                                be._p(gw), C.c_uint64(rows), C.c_uint64(dim), C.c_float(1e-6)))
+        be.silu_forward(be.upload(np.full(4, np.nan, np.float32)))  # a later op's
+        form()
+        with pytest.raises(OjasError) as e:
+            be.sync()
+        assert e.value.detail == "rms_norm_backward"
     finally:
         be.close()

@@ -711,7 +711,8 @@ def test_f32_activation_in_the_store_pass_is_named_as_the_separate_pass_is(be, t
 def test_both_gradients_in_one_launch(be, pair, rows, kin, nout):
     """Each pair of tiles, forced where it fits, and the rule's choice: outputs that end inside a tile, walks of one step, of fewer
     steps than waves and ending inside one, more tiles than compute units; against the f64 products, k products and k sums rounded
-    to f32 each: (k + 1) 2^-24 sum |a||b|. A value that is not finite is named; outputs that overlap an operand take two launches."""
+    to f32 each: (k + 1) 2^-24 sum |a||b|. A value that is not finite is named; outputs that overlap an operand take two launches.
+    The weight gradient has an order of sums of its own there, no further from the f64 product than a call's for it alone."""
     from ojas_amd.backend import OjasError
 
     print(f"gradients together {pair} {rows}x{kin}x{nout}", flush=True)
@@ -722,11 +723,24 @@ def test_both_gradients_in_one_launch(be, pair, rows, kin, nout):
     bounds = [(nout + 1) * 2.0 ** -24 * (np.abs(g64) @ np.abs(w64)), (rows + 1) * 2.0 ** -24 * (np.abs(g64).T @ np.abs(x64))]
     dx, dw, dg = (be.upload(a) for a in (x, w, gy))
     be.set_option("gemm_f32_pair", pair)
+    launches = C.c_uint64()
+
+    def launched(call):
+        be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(1)))
+        result = call()
+        be._check(be._lib.omx_profile_gemm_report(be._ctx, C.byref(launches), None, None))
+        be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(0)))
+        return launches.value, result
+
     try:
-        for got, want, bound in zip(be.linear_backward(dx, dw, dg), (g64 @ w64, g64.T @ x64), bounds):
+        count, grads = launched(lambda: be.linear_backward(dx, dw, dg))
+        assert count == 1 or (pair < 0 and rows not in (700, 900, 500))
+        for got, want, bound in zip(grads, (g64 @ w64, g64.T @ x64), bounds):
             assert (np.abs(be.download(got) - want) <= bound + 1e-30).all()
         if pair < 0:  # the input gradient's bits do not depend on who asks for it
             assert np.array_equal(be.download(be.linear_backward(dx, dw, dg)[0]), be.download(be.linear_backward_input(dw, dg)))
+            off = [np.linalg.norm(be.download(g) - g64.T @ x64) for g in (grads[1], be.linear_backward(dx, dw, dg, need_gx=False)[1])]
+            assert off[0] <= 1.05 * off[1], off
         before = r.normal(size=x.shape).astype(np.float32)
         onto, gw = be.linear_backward_onto(be.upload(before), dx, dw, dg)
         assert (np.abs(be.download(onto) - (g64 @ w64 + before)) <= bounds[0] * (nout + 2) / (nout + 1) + 2.0 ** -23 * np.abs(before)).all()
@@ -739,7 +753,7 @@ def test_both_gradients_in_one_launch(be, pair, rows, kin, nout):
         apart = be.download(gw)
         dx = be.upload(x)
         be.set_option("gemm_f32_pair", pair)
-        back(dx)
+        assert launched(lambda: back(dx))[0] == 2
         assert np.array_equal(be.download(gw), apart)
         gy[-1, -1] = np.inf
         be.linear_backward(be.upload(x), dw, be.upload(gy))
