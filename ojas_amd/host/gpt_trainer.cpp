@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "ojas_gpt.h"
+#include "waiting_sums.h"
 
 namespace {
 
@@ -214,20 +215,6 @@ int32_t forward(ogpt* t) {
   }
   return OMX_OK;
 }
-
-// Weight gradients of the norms wait for one launch (omx_defer_weight_sums); forgotten where the backward ends early.
-struct WaitingSums {
-  omx_ctx* ctx;
-  bool formed = false;
-  WaitingSums(omx_ctx* c, uint32_t count) : ctx(c) { (void)omx_defer_weight_sums(ctx, count); }
-  ~WaitingSums() {
-    if (!formed) (void)omx_form_weight_sums(ctx, 0);
-  }
-  int32_t form() {
-    formed = true;
-    return omx_form_weight_sums(ctx, 1);
-  }
-};
 
 int32_t backward(ogpt* t) {
   omx_ctx* ctx = t->ctx;

@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "ojas_nanolab.h"
+#include "waiting_sums.h"
 
 namespace {
 
@@ -236,21 +237,6 @@ int32_t forward(onano* t) {
   }
   return OMX_OK;
 }
-
-// Weight gradients of the norms and bias gradients of the gates wait for one launch (omx_defer_weight_sums); forgotten where the
-// backward ends early.
-struct WaitingSums {
-  omx_ctx* ctx;
-  bool formed = false;
-  WaitingSums(omx_ctx* c, uint32_t count) : ctx(c) { (void)omx_defer_weight_sums(ctx, count); }
-  ~WaitingSums() {
-    if (!formed) (void)omx_form_weight_sums(ctx, 0);
-  }
-  int32_t form() {
-    formed = true;
-    return omx_form_weight_sums(ctx, 1);
-  }
-};
 
 int32_t backward(onano* t, float loss_seed) {
   omx_ctx* ctx = t->ctx;
