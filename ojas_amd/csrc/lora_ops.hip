@@ -116,9 +116,11 @@ __global__ void rope_pitched_out_kernel(const TIN* __restrict__ x, unsigned shor
 }
 
 // Bytes of gate_up from which it is read past the caches: in the forward, right after the product that wrote it, where the memory-side
-// cache holds little of it; in the backward where that has forgotten it. 8192 x 2 x 8192 f32 (512 MiB): forward 144.6 -> 111.8 us,
-// backward 162.1 -> 146.6; 16384 x 2 x 2048 (256 MiB): forward 59.5, 61.8 with the hint, backward 83.2 -> 72.4.
-constexpr uint64_t SWIGLU_FWD_STREAM = 384ull << 20, SWIGLU_BWD_STREAM = 128ull << 20;
+// cache does not hold all of it; in the backward, a step's other layers after the forward, where that has forgotten it. us, without and
+// with the hint, f32, hidden 2048 / 8192: forward behind its product 192 MiB 36, 41 / 37, 40; 256 56, 62 / 57, 66; 288 80, 68 / 77, 64; 320
+// 87, 66 / 86, 65; 512 142, 101 / 125, 92. Backward: steps of six 2048 -> 8192 layers, 106 MiB 7224, 7152; 128 8049, 7927; 162 9917, 9850.
+// (The backward over and over, its tensors where it left them: 128 MiB 33, 38; 192 60, 56; 512 160, 144.)
+constexpr uint64_t SWIGLU_FWD_STREAM = 288ull << 20, SWIGLU_BWD_STREAM = 128ull << 20;
 
 // gate_up: [rows][2 * hidden] (gate columns first), bf16 or f32 (the projection's output as its
 // product left it, so the activation is rounded once, when it is stored as the next product's

@@ -37,7 +37,8 @@ def test_adamw_over_a_large_arena(be, n):
     assert whole[0].dtype == F32
 
 
-@pytest.mark.parametrize("rows,hidden,bf16", [(8192, 6144, False), (8192, 6152, False), (12288, 8192, True)])
+@pytest.mark.parametrize("rows,hidden,bf16", [(8192, 6144, False), (8192, 6152, False), (12288, 8192, True), (8192, 4608, False),
+                                              (8192, 4600, False)])  # last: the first size whose forward is streamed, and one under it
 def test_swiglu_over_a_large_projection(be, rows, hidden, bf16):
     from ojas_amd.backend import BF16, F32
 
