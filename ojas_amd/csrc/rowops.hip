@@ -874,14 +874,13 @@ int32_t omx_form_sums(omx_ctx* ctx) {
   return OMX_OK;
 }
 
-// The rows are those of the wide kernel, whose order the list keeps. Full memory is formed and used again. Rows of more than 1 MiB
-// are added at once: 16384 rows of 768 leave 1.5 MiB a norm, and the step that makes 25 of them, whose clock its products hold down,
-// took 18.26 ms with one launch for all where it takes 18.22 with one each.
+// The rows are those of the wide kernel, whose order the list keeps. Full memory is formed and used again. (Rows of more than 1 MiB
+// too: 16384 rows of 768 leave 1.5 MiB a norm, and the step that makes 25 of them takes 18.03 ms, 18.11 with a launch for each; with
+// 8192 rows 11.44 and 11.51, with gates 26.06 and 26.19. Three runs of each, in turn; those of one side are within 0.06.)
 float* omx_partial_rows(omx_ctx* ctx, uint64_t blocks, uint64_t dim) {
   if (!ctx->sums_wait || blocks <= 16 || blocks > OMX_COLUMN_SUM_WIDE_ROWS) return nullptr;
   constexpr uint64_t kMost = 64ull << 20;
   const uint64_t bytes = (blocks * dim * sizeof(float) + 255) / 256 * 256;
-  if (bytes > 1ull << 20) return nullptr;
   if (ctx->sums_used + bytes > ctx->workspace_bytes[kSumsSlot] && omx_form_sums(ctx) != OMX_OK) return nullptr;
   const uint64_t held = ctx->workspace_bytes[kSumsSlot];
   uint64_t want = held >= ctx->sums_used + bytes ? held : std::max(bytes, std::min(kMost, bytes * ctx->sums_expected));
