@@ -625,9 +625,13 @@ int32_t launch_kv_write(omx_ctx* ctx, const KvWrite& w) {
   return OMX_OK;
 }
 
-// Bytes of keys and values from which a call reads them past the caches: half of the memory-side cache, of which a model of two layers
-// and more leaves nothing for the next token. 12 layers, us a call, without and with the hint: 64 x 12 heads x 1024 f32 positions (403 MB)
-// 73.1, 66.4; bf16 (201 MB) 47.3, 45.2; two layers of 118 MB, which stay in the cache, 23.1 and 25.0.
+// Bytes of keys and values from which a call reads them past the caches: half of the memory-side cache, of which a model, with its
+// weights, leaves nothing for the next token. Whole steps of d = 768 over 1024 positions, us without and with the hint: twelve layers of
+// 126 MiB (f32) 2107, 2108; 138 MiB 2159, 2132; 150 2183, 2142; of 129 MiB (bf16) 2222, 2200; two layers of 126 MiB 448, 444; 138 462, 450;
+// one layer of 144 MiB 278, 282; 180 285, 284 (three runs of each, within 2 % at two layers and fewer). The call alone, in turn over twelve
+// caches: 144 MiB 37.9, 35.7; 384 (64 sequences) 75.0, 68.1; bf16 129 MiB 39.3, 37.1; 192 48.2, 45.3. Left: one cache over and over with
+// nothing else read in between, which stays up to its size: f32 144 MiB 30.5, 33.2; 240 42.7, 46.6; 318 62.3, 58.7; two in turn, bf16 129
+// MiB 35.1, 36.7; 144 38.1, 37.3.
 constexpr uint64_t KV_STREAM = 128ull << 20;
 template <typename T, int LPK, int NPL>
 int32_t launch_group(omx_ctx* ctx, const KvArgs& a, dim3 grid, long rows_total, int waves) {

@@ -19,7 +19,9 @@ namespace {
 
 constexpr int OPT_THREADS = 256;
 // Bytes of parameters, gradients and moments from which AdamW reads and writes them past the caches, which a step between two
-// updates has long filled with other things: 124.4 M parameters 682 -> 585 us (6.4 TB/s), 35.5 M 174 -> 156.
+// updates has long filled with other things: 124.4 M parameters inside their step 696 -> 649 us (5.7 TB/s), 35.5 M 186 -> 158. Alone,
+// behind 1 GiB of other reads and writes, us without and with the hint: 192 MiB 109, 109; 256 146, 142; 384 213, 206; 1024 556, 514; one
+// update straight after another, whose tensors partly stay, 256 MiB 118, 123; 320 170, 157; 512 291, 247.
 constexpr uint64_t OPT_STREAM = 256ull << 20;
 
 struct AdamWords {
