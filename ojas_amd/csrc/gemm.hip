@@ -505,8 +505,8 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 }  // namespace
 
-// Both gradients of an f32 linear layer in one launch where that is estimated to take less (259 layers of
-// 24 .. 6000 rows and 12 .. 1600 columns: 4.44 -> 3.80 ms of calls in all, the three it lost on 5, 6 and 12 % slower; 157 of whole
+// Both gradients of an f32 linear layer in one launch where that is estimated to take less (250 such layers of 24 .. 6000 rows and
+// 12 .. 1600 columns: 3.32 -> 2.55 ms of calls in all, none over 3 % slower; 157 of whole
 // steps, where gx takes the direct-to-LDS form: 4.13 -> 3.66, one 8 % slower). gx has the bits of a call that asks for it alone: the
 // form is the one of f32_tile's choice for it, with the estimate of the 32 x 32 pair for the direct-to-LDS ones (at 1.1 and 1.25
 // of the two apart, 5 and 11 of the 157 lost). gw's sums, folded every 16 rows on eight waves, have another order than a call's for

@@ -228,8 +228,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_frag32_kernel(GemmArgs g) {
 // A layer some hundred wide gives each of its two gradients less than a workgroup per compute unit or little more, and a call of the
 // two a fixed part of some 3 us twice and two part-empty rounds: their tiles go out together. w: both operands k-major, usually the
 // longer walk, so its workgroups come first; x: behind them, from workgroup `x_first` (a multiple of 8). x's sums are those of gemm_frag32_kernel's eight waves, whatever the tile: an
-// input gradient's bits are the same from a call that asks for it alone. w's fold every 16 values (frag32_sums). A call of both with
-// its host part: 1024 rows, 256 -> 256 11.1 -> 7.1 us, 256 -> 128 10.3 -> 6.4, 256 -> 12 9.5 -> 6.0; bound as gemm_frag32_kernel.
+// input gradient's bits are the same from a call that asks for it alone. w's fold every 16 values (frag32_sums). Kernel time of a
+// call of both: 1024 rows, 256 -> 256 10.6 -> 8.1 us, 256 -> 128 9.6 -> 6.9, 256 -> 12 9.4 -> 5.7 (9.2 and 7.8 for the first two inside a
+// step, whose operands are further away); bound as gemm_frag32_kernel.
 constexpr int PAIR_WAVES = 8;
 template <int XM, int XN, int WM, int WN>
 __global__ __launch_bounds__(PAIR_WAVES * 64) void gemm_frag32_pair_kernel(GemmArgs x, GemmArgs w, int x_first) {
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(PAIR_WAVES * 64) void gemm_frag32_pair_kernel(GemmA
 }
 
 // The same where the input gradient alone would run on gemm_dma32_kernel with KG groups of waves: its sums, on eight waves. 1024 rows,
-// 256 -> 704 16.7 -> 13.2 us a call, 704 -> 256 18.2 -> 14.4; 512 rows of 512 -> 512 13.0 -> 9.9.
+// 256 -> 704 17.2 -> 12.2 us, 704 -> 256 17.7 -> 13.8; 512 rows of 512 -> 512 12.7 -> 9.2.
 template <int KG>
 struct PairDma;  // waves of a group, blocks of a wave
 template <> struct PairDma<1> { static constexpr int WGM = 4, WGN = 2, TM = 1, TN = 2; };
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(PAIR_WAVES * 64) void gemm_dma32_pair_kernel(GemmAr
 // in one launch each; bound by the waits of short walks over K (a third of the f32 matrix rate). 64 x 32 tiles took 22, 16 and 30,
 // steps of 32 K values with all of a step's loads together 28, 16 and 33. The third products, whose outputs are the matrices, go on
 // gemm_dma32.hip's 64 x 64 tiles instead where those make half a workgroup per compute unit (28 -> 23 us: half the operand bytes a
-// product; a step of the 32 matrices 337 -> 308 us, of 64 556 -> 508, 16 matrices 240 -> 237).
+// product; a step of the 32 matrices 337 -> 305 us, of 64 556 -> 502, 16 matrices 240 -> 231).
 // `symmetric`: the output equals its transpose (X X^T, A A and their sums with a symmetric tensor): tiles below the diagonal are
 // written from those above it, the same sums in the same order.
 constexpr int GROUP_WAVES = 4, GROUP_TILE = 32, GROUP_DMA = 4, GROUP_DMA_TILE = 64;

@@ -465,8 +465,8 @@ int32_t muon_batch(omx_ctx* ctx, const char* op, void* const* params, const void
 // Whether a shape's products go out with other shapes': f32 with the sums in the store passes, operands whose rows the group's tiles can
 // read (widths in multiples of four), and at most MU_TOGETHER multiplications a product, its batch in all: there a launch's fixed time
 // is worth more than the larger tiles that a launch of its own would take. A model's step, us, a set of launches for each shape / one
-// for those that go together: 4 blocks of d = 128 419 / 129, of 256 620 / 346, of 384 1125 / 1022 (1125 with half the limit), of 512
-// 1689 / 1601 (1629).
+// for those that go together (with half the limit): 4 blocks of d = 128 413 / 134, of 256 586 / 305, 8 of 256 767 / 502 (588), 4 of 384
+// 1190 / 891 (1004), of 512 1686 / 1565 (1631).
 constexpr uint64_t MU_TOGETHER = 1ull << 30;
 bool goes_together(omx_ctx* ctx, uint64_t rows, uint64_t cols, uint64_t count, bool bf16) {
   if (bf16 || !ctx->muon_fused_sums || ctx->gemm_dma_mode != 1 || ctx->gemm_f32_tile >= 0 /* a forced kernel or tile */ || rows % 4 != 0 || cols % 4 != 0 || rows > 1u << 15 || cols > 1u << 15) return false;
