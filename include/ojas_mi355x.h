@@ -741,7 +741,8 @@ int32_t omx_profile_gemm_report(omx_ctx* ctx, uint64_t* launches, double* total_
  * forward, 2 flash attention backward (mean key row, dQ, dK / dV kernels as one
  * launch), 3 the fused cross-entropy row kernel, 4 AdamW (checking pass, when
  * it runs, and update), 5 RMSNorm forward and 6 backward (with the weight
- * gradient's column sum) for row widths 256..2048, 7 embedding backward (count,
+ * gradient's column sum; the launch that forms those that waited is one of its
+ * own) for row widths 256..2048, 7 embedding backward (count,
  * scan, fill, sort and accumulate kernels as one launch). A launch's work is
  * its algorithmic FLOPs (classes 0..2: 2 B H T^2 D forward and 5 B H T^2 D
  * backward, causal-counted) or its algorithmic bytes (classes 3..7: every

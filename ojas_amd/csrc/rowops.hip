@@ -868,7 +868,9 @@ int32_t omx_form_sums(omx_ctx* ctx) {
       list.of[i] = sums[first + i];
       dim = std::max(dim, list.of[i].dim);
     }
-    omx_launch(ctx, column_sum_list_kernel, dim3((dim + 63) / 64, static_cast<unsigned>(count)), dim3(1024), 0, list, ctx->fault);
+    OmxKernelTimer timer(ctx, OMX_K_RMS_BWD, 0.0);  // (the norms' own launches count the bytes)
+    omx_launch_timed(ctx, column_sum_list_kernel, dim3((dim + 63) / 64, static_cast<unsigned>(count)), dim3(1024), 0, timer.start(), timer.stop(),
+                     list, ctx->fault);
     OMX_LAUNCH_CHECK(ctx, "column_sum_list_kernel");
   }
   return OMX_OK;

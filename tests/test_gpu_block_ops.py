@@ -827,6 +827,14 @@ def test_a_sum_that_waits_is_formed_before_anyone_could_miss_it():
 
         form = lambda how: be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(how)))
         assert np.array_equal(be.download(wait()), want)
+        launches, ms = C.c_uint64(), C.c_double()
+        be._check(be._lib.omx_profile_kernels(be._ctx, C.c_uint32(1 << 6)))
+        timed = wait()
+        form(1)
+        be._check(be._lib.omx_profile_kernels_report(be._ctx, C.c_int32(6), C.byref(launches), C.byref(ms), None))
+        be._check(be._lib.omx_profile_kernels(be._ctx, C.c_uint32(0)))
+        assert launches.value == 2 and ms.value > 0  # the norm, and the launch that forms its sum
+        assert np.array_equal(be.download(timed), want)
         first = wait()
         second = wait()
         form(0)
