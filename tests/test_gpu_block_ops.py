@@ -912,3 +912,28 @@ def test_gate_bias_sums_wait_and_overflows_are_named():
         assert e.value.detail == "rms_norm_backward"
     finally:
         be.close()
+
+
+@pytest.mark.parametrize("rows,dim", [(8192, 2048), (16384, 768), (16380, 512)])
+def test_weight_sums_over_a_large_batch_wait_too(rows, dim):
+    """1.5 MiB of partial rows and more a norm, three of them in one launch: the bits of a launch for each."""
+    from ojas_amd.backend import F32, MiBackend
+
+    print(f"weight sums {rows}x{dim}", flush=True)
+    rng = np.random.default_rng(dim)
+    be = MiBackend(0)
+    try:
+        x, gy = (be.upload(rng.standard_normal((rows, dim), dtype=np.float32)) for _ in range(2))
+        ws = [be.upload(rng.normal(1, 0.1, dim).astype(np.float32)) for _ in range(3)]
+        want = [be.download(be.rms_norm_backward(x, w, gy, 1e-6)[1]) for w in ws]
+        got, gx, before = [be.zeros((dim,)) for _ in ws], be.empty((rows, dim), F32), be.empty((dim,), F32)
+        be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(3)))
+        for w, gw in zip(ws, got):
+            be._check(be._lib.omx_rms_norm_backward(be._ctx, be._p(x), C.c_int32(F32), be._p(w), be._p(gy), C.c_int32(F32), be._p(gx), C.c_int32(F32),
+                                                    be._p(gw), C.c_uint64(rows), C.c_uint64(dim), C.c_float(1e-6)))
+        be._check(be._lib.omx_copy(be._ctx, be._p(before), be._p(got[0]), C.c_uint64(before.nbytes)))
+        be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
+        assert all(np.array_equal(be.download(a), b) for a, b in zip(got, want))
+        assert not be.download(before).any()
+    finally:
+        be.close()
