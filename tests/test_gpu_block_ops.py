@@ -916,7 +916,7 @@ def test_gate_bias_sums_wait_and_overflows_are_named():
 
 @pytest.mark.parametrize("rows,dim", [(8192, 2048), (16384, 768), (16380, 512)])
 def test_weight_sums_over_a_large_batch_wait_too(rows, dim):
-    """1.5 MiB of partial rows and more a norm, three of them in one launch: the bits of a launch for each."""
+    """1 MiB of partial rows and more a norm, three of them in one launch: the bits of a launch for each."""
     from ojas_amd.backend import F32, MiBackend
 
     print(f"weight sums {rows}x{dim}", flush=True)
