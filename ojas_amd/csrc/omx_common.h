@@ -12,7 +12,9 @@
 #include <cstring>
 #include <initializer_list>
 #include <map>
+#include <set>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "ojas_mi355x.h"
@@ -75,14 +77,21 @@ struct OmxColumnSum {
   int blocks, dim;
 };
 
+// Freed blocks of one size, kept for the next request of it; the numbers of the last two requests (omx_ctx::requests).
+struct OmxParked {
+  std::vector<std::map<void*, uint64_t>::node_type> blocks;
+  uint64_t last = 0, before = 0;
+};
+
 struct omx_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   uint64_t budget_limit = 0, budget_live = 0, budget_peak = 0;
   std::map<void*, uint64_t> allocations;
   // Freed blocks kept for reuse by size (see omx_free); not charged to the budget.
-  std::multimap<uint64_t, void*> pool;
-  uint64_t pooled_bytes = 0;
+  std::unordered_map<uint64_t, OmxParked> pool;
+  uint64_t pooled_bytes = 0, requests = 0;
+  std::set<void*> freed_in_capture;  // blocks a captured graph may still write: they stay with the context
   OmxFaultWord* fault = nullptr;  // device
   OmxFaultWord* fault_host = nullptr;  // pinned, with kReadback bytes for what a small download brings behind it
   // Pinned memory that small uploads pass through (omx_upload_staged), taken by the first; up to `staged` the stream may still read it.

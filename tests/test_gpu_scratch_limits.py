@@ -315,3 +315,49 @@ def test_sums_that_wait_make_room_for_what_is_allocated_next():
         del rest
     finally:
         be.close()
+
+
+def test_a_full_pool_makes_room_for_a_size_that_comes_back():
+    """Parked blocks of sizes no longer asked for go back to the device for one that is asked for again and again; the sizes of a
+    round through more than the pool holds stay, and so does a block that a capture freed, which its graph still writes."""
+    from ojas_amd.backend import MiBackend
+
+    be = MiBackend(0)
+    most = 4 << 30
+    x = be.upload(np.full((1 << 16,), 1.5, np.float32))
+    print("graph with a temporary", flush=True)
+    graph = Graph(be, lambda: be.residual_add_forward(be.residual_add_forward(x, x), x))
+    print("4 GiB parked", flush=True)
+    held = [be.empty(((200 << 18) + 1024 * k,)) for k in range(21)]
+    parked_first = held[0].ptr
+    del held
+    full = be.budget()["pooled"]
+    assert most - (201 << 20) < full <= most
+    held = [be.empty((n,)) for n in (1 << 25, 1 << 25)]  # up to less than 16 MiB below the limit, or nothing left to fill
+    del held
+    print("a size that comes back", flush=True)
+    n = (200 << 18) - 1024
+    seen = []
+    for _ in range(4):
+        t = be.empty((n,))
+        seen.append(be.budget()["pooled"])
+        del t
+        assert be.budget()["pooled"] <= most
+    assert seen[3] == be.budget()["pooled"] - 4 * n, "the fourth was not taken from the pool"
+    for _ in range(3):
+        graph.launch()
+        assert np.array_equal(be.download(graph.results), np.full((1 << 16,), 4.5, np.float32))
+    assert parked_first
+    print("a round through more than the pool holds", flush=True)
+    sizes = [(160 << 18) + 1024 * k for k in range(32)]
+    hits = 0
+    for turn in range(3):
+        held = []
+        for m in sizes:
+            before = be.budget()["pooled"]
+            held.append(be.empty((m,)))
+            hits += turn == 2 and be.budget()["pooled"] < before
+        del held
+    assert hits >= 20, "the pool gave up blocks that were about to be asked for"
+    graph.close()
+    be.close()
