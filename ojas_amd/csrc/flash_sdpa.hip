@@ -24,6 +24,7 @@
 //     swapped), so one 16-byte LDS read fetches exactly those rows.
 #include "omx_common.h"
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -54,6 +55,7 @@ struct FlashShape {
   // forward and dQ; key side: dK/dV). Chosen by the host when the pairs would leave workgroup
   // places empty (few planes) or, on the key side, need a half-empty second round.
   int q_single, kv_single;
+  int kv_parts;  // dK/dV: workgroups that share a key block's query tiles
   float scale;
   FlashStrides q, kv, o;  // q and grad_q; k, v and their gradients; out and grad_out
 };
@@ -639,13 +641,15 @@ __device__ __forceinline__ void flash_dkv_tile(const char* q_rows, const char* g
 // fragments (64) and the score tiles do not fit the 256 registers of two waves per SIMD, so the
 // block is walked twice, once per gradient; the second walk recomputes the scores.
 // GROUPS > 1: groups of the waves take the query tiles of 128 / GROUPS keys in turn, as in the forward.
-template <int D, typename TO, bool WANT_DK, bool WANT_DV, bool WIN, int GROUPS>
+// SPLIT: the tiles of s.kv_parts workgroups are consecutive shares of the sequence over the heads, this one's is `part`, and its sums go
+// out as rows of gk and gv, each [part][b, KV head][time][D].
+template <int D, typename TO, bool WANT_DK, bool WANT_DV, bool WIN, int GROUPS, bool SPLIT>
 __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict__ q,
                                                 const unsigned short* __restrict__ k,
                                                 const unsigned short* __restrict__ v, const float* __restrict__ lse,
                                                 const float* __restrict__ delta, const unsigned short* __restrict__ gy,
                                                 TO* __restrict__ gk, TO* __restrict__ gv, const FlashShape& s, char* lds,
-                                                int kb, int b, int gidx) {
+                                                int kb, int b, int gidx, int part) {
   constexpr int NT = FT / GROUPS, ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;
   constexpr int KK = D / 16, MT = D / 32, NL = 8 * D / NT;
   constexpr int SET = flash_dkv_set(D);
@@ -673,11 +677,15 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
   // One flat sequence of (query head of the group, query tile), ascending, so the
   // next tile's global loads can be in flight while the current one is multiplied.
   const int nq = qt_last - qt_first + 1;
-  const int steps = (s.rep * nq - group + GROUPS - 1) / GROUPS;  // this group's: GROUPS tiles apart
+  // The workgroup's tiles (none of a late key block's may be left for a late part: its sums are zeros then).
+  const int share_at = SPLIT ? static_cast<int>(static_cast<long>(s.rep) * nq * part / s.kv_parts) : 0;
+  const int share = (SPLIT ? static_cast<int>(static_cast<long>(s.rep) * nq * (part + 1) / s.kv_parts) : s.rep * nq) - share_at;
+  const int r_first = SPLIT ? share_at / nq : 0, qt_start = SPLIT ? qt_first + share_at % nq : qt_first;
+  const int steps = (share - group + GROUPS - 1) / GROUPS;  // this group's: GROUPS tiles apart
   u32x4 rq[NL], rg[NL];
   float row_lse = 0.0f, row_del = 0.0f;
   // (head of the group, query tile) of the tile being fetched.
-  int fetch_r = 0, fetch_qt = qt_first;
+  int fetch_r = r_first, fetch_qt = qt_start;
   auto skip = [&](int& r, int& qt, int tiles) {
 #pragma unroll
     for (int i = 0; i < tiles; ++i)
@@ -690,7 +698,7 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     for (int i = 0; i < group; ++i) skip(fetch_r, fetch_qt, 1);
   }
   auto fetch = [&]() {
-    const int r = GROUPS == 1 ? fetch_r : min(fetch_r, s.rep - 1), q0 = fetch_qt * 64;
+    const int r = GROUPS == 1 && !SPLIT ? fetch_r : min(fetch_r, s.rep - 1), q0 = fetch_qt * 64;
     skip(fetch_r, fetch_qt, GROUPS);
     const long q_plane = static_cast<long>(b) * s.heads + static_cast<long>(gidx) * s.rep + r;
     const long head = static_cast<long>(gidx) * s.rep + r;
@@ -740,19 +748,21 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     flash_dkv_tile<D, WANT_DK, WANT_DV, decltype(general)::value>(q_rows, g_rows, lse_s, del_s, kf, vf, dk, dv, scale_log2, q0,
                                                                  key_row, T, s.window, lane, cut);
   };
-  if constexpr (GROUPS > 1) {
-    int r = 0, qt = qt_first;
+  if constexpr (GROUPS > 1 || SPLIT) {
+    int r = r_first, qt = qt_start;
     for (int i = 0; i < group; ++i) skip(r, qt, 1);
-    const int rounds = (s.rep * nq + GROUPS - 1) / GROUPS;
+    const int rounds = (share + GROUPS - 1) / GROUPS;
     for (int i = 0; i < rounds; ++i) {
       advance();
       const int q0 = qt * 64;
-      if (r < s.rep && wave_k0 < T && q0 + 63 >= wave_k0 && (!WIN || q0 < wave_k0 + 31 + s.window)) {
+      if ((SPLIT ? i * GROUPS + group < share : r < s.rep) && wave_k0 < T && q0 + 63 >= wave_k0 && (!WIN || q0 < wave_k0 + 31 + s.window)) {
         if constexpr (WIN) tile(std::true_type{}, q0);
         else tile(std::integral_constant<int, 2>{}, q0, q0 < wave_k0 + 32 || q0 + 64 > T || wave_k0 + 31 >= T);
       }
       skip(r, qt, GROUPS);
     }
+  }
+  if constexpr (GROUPS > 1) {
     constexpr int PART = ((WANT_DK ? MT : 0) + (WANT_DV ? MT : 0)) * 16 * 64;  // floats of a wave
     float* const meet = reinterpret_cast<float*>(lds);
     __syncthreads();  // every wave is done with the tiles
@@ -780,7 +790,7 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
         }
     }
   }
-  for (int r = 0; GROUPS == 1 && r < s.rep; ++r) {
+  for (int r = 0; GROUPS == 1 && !SPLIT && r < s.rep; ++r) {
     int qt = qt_first;
     if constexpr (WIN) {
       for (; qt <= qt_last; ++qt) {
@@ -809,12 +819,13 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     }
     for (; qt <= qt_last; ++qt) advance();
   }
-  if constexpr (WANT_DK) bad |= store_transposed_acc<D, TO>(gk + kv_off, s.kv.rs, key_row, T, lg, dk, s.scale);
-  if constexpr (WANT_DV) bad |= store_transposed_acc<D, TO>(gv + kv_off, s.kv.rs, key_row, T, lg, dv, 1.0f);
+  const long out_off = SPLIT ? ((static_cast<long>(part) * s.batch + b) * s.kv_heads + gidx) * T * D : kv_off, out_rs = SPLIT ? D : s.kv.rs;
+  if constexpr (WANT_DK) bad |= store_transposed_acc<D, TO>(gk + out_off, out_rs, key_row, T, lg, dk, s.scale);
+  if constexpr (WANT_DV) bad |= store_transposed_acc<D, TO>(gv + out_off, out_rs, key_row, T, lg, dv, 1.0f);
   return bad;
 }
 
-template <int D, typename TO, bool WIN, int GROUPS>
+template <int D, typename TO, bool WIN, int GROUPS, bool SPLIT>
 __global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_dkv_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const float* __restrict__ lse, const float* __restrict__ delta, const unsigned short* __restrict__ gy,
@@ -825,9 +836,14 @@ __global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_dkv_
   // Early key blocks are seen by the most queries: a workgroup takes one of them and then its
   // mirror image from the back (see the forward kernel).
   const int k_blocks = (s.time + 128 / GROUPS - 1) / (128 / GROUPS);
-  int pair;
+  int pair, part = 0;
   long kv_plane;
-  if (s.kv_single) {  // block index (0 = the first, heaviest block) in the high part of the index
+  if constexpr (SPLIT) {  // (one block per workgroup)
+    const int planes = s.batch * s.kv_heads, rest = static_cast<int>(blockIdx.x) % (planes * s.kv_parts);
+    pair = static_cast<int>(blockIdx.x) / (planes * s.kv_parts);
+    part = rest / planes;
+    kv_plane = rest % planes;
+  } else if (s.kv_single) {  // block index (0 = the first, heaviest block) in the high part of the index
     pair = static_cast<int>(blockIdx.x) / (s.batch * s.kv_heads);
     kv_plane = static_cast<int>(blockIdx.x) % (s.batch * s.kv_heads);
   } else {
@@ -835,17 +851,45 @@ __global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_dkv_
   }
   const int gidx = static_cast<int>(kv_plane % s.kv_heads), b = static_cast<int>(kv_plane / s.kv_heads);
   bool bad = false;
-  for (int pass = 0; pass < (s.kv_single ? 1 : 2); ++pass) {
+  for (int pass = 0; pass < (SPLIT || s.kv_single ? 1 : 2); ++pass) {
     const int kb = pass == 0 ? pair : k_blocks - 1 - pair;
     if (pass == 1 && kb <= pair) break;
     if constexpr (D == 64) {
-      bad |= flash_dkv_block<D, TO, true, true, WIN, GROUPS>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
+      bad |= flash_dkv_block<D, TO, true, true, WIN, GROUPS, SPLIT>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx, part);
     } else {
-      bad |= flash_dkv_block<D, TO, false, true, WIN, GROUPS>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
-      bad |= flash_dkv_block<D, TO, true, false, WIN, GROUPS>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx);
+      bad |= flash_dkv_block<D, TO, false, true, WIN, GROUPS, SPLIT>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx, part);
+      bad |= flash_dkv_block<D, TO, true, false, WIN, GROUPS, SPLIT>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx, part);
     }
   }
   if (bad) dev_raise_fault(fault, tag);
+}
+
+// Adds up the parts of a split dK/dV pass, first tiles first: 8 values of a row a thread. blockIdx.y: 0 dK, 1 dV.
+template <int D, typename TO>
+__global__ __launch_bounds__(256) void flash_parts_kernel(const float* __restrict__ parts, TO* __restrict__ gk, TO* __restrict__ gv,
+                                                          FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
+  const long total = static_cast<long>(s.batch) * s.kv_heads * s.time * D, at = (static_cast<long>(blockIdx.x) * 256 + threadIdx.x) * 8;
+  if (at >= total) return;
+  const float* src = parts + static_cast<long>(blockIdx.y) * s.kv_parts * total + at;
+  float4 lo = *reinterpret_cast<const float4*>(src), hi = *reinterpret_cast<const float4*>(src + 4);
+#pragma unroll 4
+  for (int z = 1; z < s.kv_parts; ++z) {
+    const float4 l = *reinterpret_cast<const float4*>(src + z * total), h = *reinterpret_cast<const float4*>(src + z * total + 4);
+    lo.x += l.x; lo.y += l.y; lo.z += l.z; lo.w += l.w;
+    hi.x += h.x; hi.y += h.y; hi.z += h.z; hi.w += h.w;
+  }
+  const long row = at / D, plane = row / s.time, b = plane / s.kv_heads;
+  TO* dst = (blockIdx.y ? gv : gk) + b * s.kv.bs + (plane - b * s.kv_heads) * s.kv.hs + (row - plane * s.time) * s.kv.rs + (at - row * D);
+  if constexpr (sizeof(TO) == 2) {
+    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(lo.x, lo.y), pack2(lo.z, lo.w));  // (8-byte rows, as the unsplit pass stores them)
+    *reinterpret_cast<uint2*>(dst + 4) = make_uint2(pack2(hi.x, hi.y), pack2(hi.z, hi.w));
+  } else {
+    *reinterpret_cast<float4*>(dst) = lo;
+    *reinterpret_cast<float4*>(dst + 4) = hi;
+  }
+  if (!(dev_finite(lo.x) && dev_finite(lo.y) && dev_finite(lo.z) && dev_finite(lo.w) && dev_finite(hi.x) && dev_finite(hi.y) &&
+        dev_finite(hi.z) && dev_finite(hi.w)))
+    dev_raise_fault(fault, tag);
 }
 
 // ------------------------------------------------------------------ backward: dQ
@@ -1132,6 +1176,7 @@ FlashShape make_shape(uint64_t batch, uint64_t heads, uint64_t kv_heads, uint64_
   s.window = static_cast<int>(window);
   s.rep = static_cast<int>(heads / kv_heads);
   s.q_single = s.kv_single = 0;
+  s.kv_parts = 1;
   s.scale = scale;
   return s;
 }
@@ -1223,6 +1268,57 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
   for_groups<D>(groups, with_groups);
 }
 
+// Into how many parts the query tiles that a key block sees are split (1: none), and the groups of waves that go with it. The pass has a
+// workgroup per key block and KV head, so few KV heads leave units idle however many query heads there are, and each workgroup walks
+// the tiles of all of them, 1.9 us apiece. A part is a consecutive share of those tiles on a workgroup of its own; its f32 sums go through
+// scratch to a second launch that adds them in order. The estimate is the root of the squares of the longest walk and of the
+// chip's work, per key block of 128 or 64 keys, fitted to 24 shapes x 3 group counts x 9 part counts; the second launch takes 4.5 us
+// or 0.13 us a megabyte. Taken where that is an eighth less, for the fit is no better (15 to 25 %).
+// us of the pass, before / now: 10 x 13 heads over one x 670: 112 / 47; 5 x 2 over 1 x 1161 x 128, window 612: 92 / 45;
+// 8 over 2 x 291 x 128: 77 / 24; 2 x 8 over 2 x 1024 x 128: 186 / 47; 15 x 14 over 2 x 122: 26 / 19; 5 x 1000 x 128: 58 / 34;
+// 4 x 4096: 56 / 44. Many planes (8 x 12 x 1024: 49, split in two 77) stay as they are.
+int flash_kv_parts(omx_ctx* ctx, const FlashShape& s, int dim, int* groups) {
+  if (ctx->flash_kv_parts) return ctx->flash_kv_parts;
+  if (ctx->flash_schedule != 0) return 1;
+  const long units = ctx->cu_count > 0 ? ctx->cu_count : 256, planes = static_cast<long>(s.batch) * s.kv_heads;
+  if (planes * ((s.time + 127) / 128) >= 2 * units) return 1;
+  struct Fit {
+    double first, step, work, each;  // us: of a workgroup, of a tile on its way; of a unit's tiles, of a unit's workgroups
+  };
+  const Fit fits[2][2] = {{{7.6, 1.9, 0.74, 4.07}, {7.66, 2.08, 0.78, 3.5}}, {{12.23, 4.74, 0.77, 10.93}, {11.53, 5.68, 2.84, 12.98}}};
+  const double megabytes = 8e-6 * static_cast<double>(planes) * s.time * dim;
+  double whole = 1e30, least = 1e30;
+  int parts = 1, by = 1;
+  for (int g = 1; g <= 2; ++g) {
+    const Fit& f = fits[dim == 128][g - 1];
+    const int rows = 128 / g, blocks = (s.time + rows - 1) / rows;
+    long all = 0, most = 0;
+    for (int kb = 0; kb < blocks; ++kb) {
+      const int last = s.window > 0 ? std::min<long>(s.time - 1, std::min(s.time - 1, kb * rows + rows - 1) + static_cast<long>(s.window) - 1) : s.time - 1;
+      const long tiles = static_cast<long>(s.rep) * (last / 64 - kb * rows / 64 + 1);
+      all += tiles;
+      most = std::max(most, tiles);
+    }
+    for (const int p : {1, 2, 3, 4, 6, 8, 12, 16, 24}) {
+      if (p > most || (p > 1 && p * megabytes > 256.0)) break;
+      const double groups_of_units = static_cast<double>(blocks * planes * p) / static_cast<double>(units);
+      const double walk = f.first + f.step * static_cast<double>((most + p * g - 1) / (p * g));
+      const double work = f.work * (static_cast<double>(all * planes) / static_cast<double>(g * units) + (p * g > 1 ? 0.5 * groups_of_units : 0.0)) + f.each * groups_of_units;
+      const double us = std::sqrt(walk * walk + work * work) + (p > 1 ? std::max(4.5, 2.5 + 0.13 * megabytes * p) : 0.0);
+      if (p == 1) {
+        whole = std::min(whole, us);
+      } else if (us < least) {
+        least = us;
+        parts = p;
+        by = g;
+      }
+    }
+  }
+  if (least >= 0.875 * whole) return 1;
+  *groups = by;
+  return parts;
+}
+
 template <int D>
 void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short* k, const unsigned short* v,
                      const unsigned short* out, const unsigned short* resid, const float* lse, float* delta,
@@ -1237,18 +1333,26 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
   const unsigned kv_planes = static_cast<unsigned>(s.batch * s.kv_heads), q_planes = static_cast<unsigned>(s.batch * s.heads);
   const int tiles = flash_tiles(s);
   const int q_groups = flash_groups(ctx, q_planes, s.time, tiles, s.window > 0, D);
-  const int kv_groups = flash_groups(ctx, kv_planes, s.time, static_cast<int>(std::min<long>(static_cast<long>(tiles) * s.rep, 1 << 20)), s.window > 0, D);
+  int kv_groups = flash_groups(ctx, kv_planes, s.time, static_cast<int>(std::min<long>(static_cast<long>(tiles) * s.rep, 1 << 20)), s.window > 0, D);
+  // Split where that takes less and there is room for the sums, in as many parts as there is room for.
+  const long kv_total = static_cast<long>(kv_planes) * s.time * D;
+  float* parts = nullptr;
+  int split_groups = kv_groups;
+  for (s.kv_parts = flash_kv_parts(ctx, s, D, &split_groups); s.kv_parts > 1; --s.kv_parts)
+    if ((parts = static_cast<float*>(omx_workspace_if_room(ctx, static_cast<uint64_t>(s.kv_parts) * kv_total * 8, kExtraSlot)))) break;
+  if (s.kv_parts > 1) kv_groups = split_groups;
   const unsigned q_rows = 128 / q_groups, kv_rows = 128 / kv_groups;
   s.q_single = q_groups > 1 || flash_single(ctx, pairs * q_planes, D == 64 ? 3 : 2, false);
   s.kv_single = kv_groups > 1 || flash_single(ctx, pairs * kv_planes, 2, true);
-  dim3 kv_grid((s.kv_single ? (s.time + kv_rows - 1) / kv_rows : pairs) * kv_planes);
+  if (s.kv_parts > 1) s.kv_single = 1;
+  dim3 kv_grid((s.kv_single ? (s.time + kv_rows - 1) / kv_rows : pairs) * kv_planes * s.kv_parts);
   dim3 q_grid((s.q_single ? (s.time + q_rows - 1) / q_rows : pairs) * q_planes);
   auto go_dq = [&](auto kernel, auto* gq_ptr) {
     omx_launch_timed(ctx, kernel, q_grid, block, 0, timer.start(), nullptr, q, k, v, out, resid, lse, delta, gy, gq_ptr, s, ctx->fault, tag);
   };
   auto go_dkv = [&](auto kernel, auto* gk_ptr, auto* gv_ptr) {
-    omx_launch_timed(ctx, kernel, kv_grid, block, 0, nullptr, timer.stop(), q, k, v, lse, delta, gy, gk_ptr, gv_ptr, s,
-                     ctx->fault, tag);
+    omx_launch_timed(ctx, kernel, kv_grid, block, 0, nullptr, s.kv_parts > 1 ? nullptr : timer.stop(), q, k, v, lse, delta, gy, gk_ptr,
+                     gv_ptr, s, ctx->fault, tag);
   };
   auto both = [&](auto* gq_ptr, auto* gk_ptr, auto* gv_ptr) {
     typedef std::remove_pointer_t<decltype(gq_ptr)> T;
@@ -1259,9 +1363,15 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
     });
     for_groups<D>(kv_groups, [&](auto count) {
       constexpr int G = decltype(count)::value;
-      if (s.window > 0) go_dkv(flash_bwd_dkv_kernel<D, T, true, G>, gk_ptr, gv_ptr);
-      else go_dkv(flash_bwd_dkv_kernel<D, T, false, G>, gk_ptr, gv_ptr);
+      float* const part_v = parts + s.kv_parts * kv_total;
+      if (s.kv_parts > 1 && s.window > 0) go_dkv(flash_bwd_dkv_kernel<D, float, true, G, true>, parts, part_v);
+      else if (s.kv_parts > 1) go_dkv(flash_bwd_dkv_kernel<D, float, false, G, true>, parts, part_v);
+      else if (s.window > 0) go_dkv(flash_bwd_dkv_kernel<D, T, true, G, false>, gk_ptr, gv_ptr);
+      else go_dkv(flash_bwd_dkv_kernel<D, T, false, G, false>, gk_ptr, gv_ptr);
     });
+    if (s.kv_parts > 1)
+      omx_launch_timed(ctx, flash_parts_kernel<D, T>, dim3(static_cast<unsigned>((kv_total / 8 + 255) / 256), 2), dim3(256), 0, nullptr,
+                       timer.stop(), static_cast<const float*>(parts), gk_ptr, gv_ptr, s, ctx->fault, tag);
   };
   if (grad_dtype == OMX_BF16)
     both(static_cast<unsigned short*>(gq), static_cast<unsigned short*>(gk), static_cast<unsigned short*>(gv));

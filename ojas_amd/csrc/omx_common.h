@@ -129,6 +129,7 @@ struct omx_ctx {
   int gemm_forced_tiling = -1;     // the tiling the first half keeps, whatever its own tile count says
   int gemm_thin = 1;         // outputs of at most 64 columns over many rows take gemm_thin_kernel
   int flash_schedule = 0;     // 0: by the chip's workgroup places; 1: one 128-row block per workgroup; 2: mirrored pairs
+  int flash_kv_parts = 0;     // workgroups that share a key block's query tiles: 0: by estimate; 1..64: always that many
   int kv_attention_mode = 0;  // 1: cached attention always takes the LDS-tiled kernel
   int adamw_trust = 1;        // 0: omx_adamw_step_bounded always runs its checking pass
   int ce_fused = 1;           // 0: linear-CE always takes the separate statistics and gradient kernels

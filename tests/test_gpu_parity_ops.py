@@ -995,6 +995,41 @@ def test_causal_sdpa_bf16_with_tiles_shared_by_groups_of_waves(be, shape, hkv, w
         be.set_option("flash_schedule", 0)
 
 
+@pytest.mark.parametrize("groups", [1, 2, 4])
+@pytest.mark.parametrize("parts", [2, 5])
+@pytest.mark.parametrize("shape,hkv,window", [((1, 8, 33, 64), 1, None), ((2, 6, 129, 64), 2, None), ((1, 4, 321, 64), 1, 40), ((1, 1, 300, 64), 1, None),
+                                              ((1, 4, 97, 128), 1, None), ((2, 4, 257, 128), 2, 65)])
+def test_causal_sdpa_bf16_with_a_key_block_s_tiles_shared_by_workgroups(be, shape, hkv, window, parts, groups):
+    """Key gradients summed over several workgroups' shares of the query tiles: shares that begin inside a head's tiles, shares without
+    a tile, the last key block's rows past the end, both gradient types, rows of several heads; then a value that is not finite."""
+    from ojas_amd.backend import BF16, OjasError
+
+    be.set_option("flash_schedule", {1: 1, 2: 3, 4: 4}[groups])
+    be.set_option("flash_kv_parts", parts)
+    try:
+        test_causal_sdpa_bf16_mfma(be, shape, hkv, window, f"{groups} groups, {parts} parts")
+        b, h, t, d = shape
+        rng = np.random.default_rng(t)
+        q, k, v, gy = (be.upload(rng.normal(size=(b, t, n, d)).astype(np.float32), BF16) for n in (h, hkv, hkv, h))
+        out, lse = be.causal_attention_forward(q, k, v, window)
+        split = be.causal_attention_backward(q, k, v, out, lse, gy, window)
+        be.set_option("flash_kv_parts", 1)
+        for a, e in zip(split, be.causal_attention_backward(q, k, v, out, lse, gy, window)):
+            a, e = be.download_f32(a), be.download_f32(e)  # (sums in another order, then one rounding: an ulp of bf16 apart)
+            assert np.max(np.abs(a - e)) <= 2.0**-7 * np.max(np.abs(e))
+        be.set_option("flash_kv_parts", parts)
+        x = np.ones((b, h, t, d), np.float32)
+        x[0, h - 1, t - 1, 3] = np.inf
+        ones = [be.upload(np.ones((b, n, t, d), np.float32), BF16) for n in (h, hkv, hkv)]
+        y, stat = be.causal_sdpa_forward(*ones, window, out_dtype=BF16)
+        be.causal_sdpa_backward(*ones, y, stat, be.upload(x, BF16), window, grad_dtype=BF16)
+        with pytest.raises(OjasError):
+            be.sync()
+    finally:
+        be.set_option("flash_schedule", 0)
+        be.set_option("flash_kv_parts", 0)
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("shared", [(0, 4, 0), (0, 0, 4), (4, 4, 4)])
 def test_causal_attention_keeps_its_accuracy_when_rows_share_a_component(be, dim, shared):

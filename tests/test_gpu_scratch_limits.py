@@ -361,3 +361,27 @@ def test_a_full_pool_makes_room_for_a_size_that_comes_back():
     assert hits >= 20, "the pool gave up blocks that were about to be asked for"
     graph.close()
     be.close()
+
+
+def test_attention_backward_without_room_for_shares_of_the_key_sums():
+    """Scratch for the sums of a key block's workgroups that the budget refuses: one workgroup walks all tiles, to the same bits as
+    where the option says so."""
+    from ojas_amd.backend import BF16, MiBackend
+
+    be = MiBackend(0, 16 << 20)
+    rng = np.random.default_rng(5)
+    q, k, v, gy = (be.upload(rng.normal(size=(1, n, 300, 64)).astype(np.float32), BF16) for n in (4, 1, 1, 4))
+    out, lse = be.causal_sdpa_forward(q, k, v, None, BF16)
+    be.set_option("flash_kv_parts", 1)
+    whole = [be.download_f32(g) for g in be.causal_sdpa_backward(q, k, v, out, lse, gy, None, BF16)]
+    be.set_option("flash_kv_parts", 5)  # 5 x 300 x 64 x 8 bytes
+    grads = [be.empty(t.shape, BF16) for t in (q, k, v)]
+    budget = be.budget()
+    held = be.empty(((budget["limit"] - budget["live"] - (1 << 19)) // 4,))
+    del grads
+    split = [be.download_f32(g) for g in be.causal_sdpa_backward(q, k, v, out, lse, gy, None, BF16)]
+    assert all(np.array_equal(a, e) for a, e in zip(split, whole))
+    del held
+    split = [be.download_f32(g) for g in be.causal_sdpa_backward(q, k, v, out, lse, gy, None, BF16)]
+    assert not all(np.array_equal(a, e) for a, e in zip(split, whole))
+    be.close()
