@@ -40,8 +40,8 @@ constexpr int fpitch(int D) { return D * 2 + 16; }      // bytes per LDS row: D 
 constexpr int ftile(int D) { return 64 * fpitch(D); }   // a 64-row tile
 constexpr int FT = 256;                                 // threads per block (4 waves of 32 rows)
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr int flash_dkv_set(int D) { return 2 * ftile(D) + 2 * 64 * 4; }
-constexpr int flash_dkv_waves(int D, int groups) { return groups == 1 || (groups == 2 && D == 64) ? 2 : 1; }
+constexpr int flash_dkv_set(int D) { return 2 * 64 * D * 2 + 2 * 64 * (D == 64 ? 16 : 4); }  // bytes: query and gradient tile, two values a row (DkvHalf)
+constexpr int flash_dkv_waves(int D, int groups) { return D == 64 && groups <= 2 ? 2 : 1; }
 // Waves per SIMD the query-side passes are compiled for: what their LDS leaves room for.
 constexpr int flash_waves(int D, int groups) { return groups == 1 ? (D == 64 ? 3 : 2) : groups == 2 && D == 64 ? 2 : 1; }
 
@@ -55,11 +55,21 @@ struct FlashShape {
   // forward and dQ; key side: dK/dV). Chosen by the host when the pairs would leave workgroup
   // places empty (few planes) or, on the key side, need a half-empty second round.
   int q_single, kv_single;
+  int aligned;   // q, k, v, gradients of the output: all rows 16-byte aligned
   int kv_parts;  // dK/dV: workgroups that share a key block's query tiles
   float scale;
   FlashStrides q, kv, o;  // q and grad_q; k, v and their gradients; out and grad_out
 };
 
+
+// f(integral_constant<int, i>) for i = 0 .. N - 1.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void for_sequence(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    for_sequence<N, I + 1>(f);
+  }
+}
 
 __device__ __forceinline__ unsigned int pack2(float a, float b) {
   floatx2 f = {a, b};
@@ -198,15 +208,13 @@ __device__ __forceinline__ u32x4 frag_tr(const char* lds, int mt, int sub, int c
   const u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
   return u32x4{a.x, a.y, b.x, b.y};
 }
-// B operand held in registers: the lane's own row of a [time, D] plane.
+// B operand held in registers: the lane's own row of a [time, D] plane (past its end the last one: what comes of it is masked or not stored).
 template <int D>
 __device__ __forceinline__ void row_frags(const unsigned short* __restrict__ plane, long rs, int row, int time, int lg,
                                           u32x4 (&f)[D / 16]) {
+  const unsigned short* at = plane + static_cast<long>(min(row, time - 1)) * rs + lg * 8;
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk) {
-    f[kk] = u32x4{0u, 0u, 0u, 0u};
-    if (row < time) f[kk] = *reinterpret_cast<const u32x4*>(plane + static_cast<long>(row) * rs + kk * 16 + lg * 8);
-  }
+  for (int kk = 0; kk < D / 16; ++kk) f[kk] = *reinterpret_cast<const u32x4*>(at + kk * 16);
 }
 // Row index (within a 32-row sub-tile) that accumulator register v of this lane holds.
 __device__ __forceinline__ int acc_row(int v, int lg) { return 8 * (v >> 2) + 4 * lg + (v & 3); }
@@ -573,197 +581,385 @@ __global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_fwd_kernel(c
 }
 
 // ------------------------------------------------------------------ backward: dK, dV
-// One 64-query x 32-key tile of one wave in the dK/dV pass. GENERAL: the tile crosses the diagonal,
-// the sequence end or a window edge and every element is tested (as in the dQ pass, the cheaper
-// forms of the cut tile would push the kernel past its registers): 0 / 1: no / yes, 2: as `cut` says.
-template <int D, bool WANT_DK, bool WANT_DV, int GENERAL>
-__device__ __forceinline__ void flash_dkv_tile(const char* q_rows, const char* g_rows, const float* lse_s,
-                                               const float* del_s, const u32x4 (&kf)[D / 16],
-                                               const u32x4 (&vf)[WANT_DK ? D / 16 : 1], floatx16 (&dk)[WANT_DK ? D / 32 : 1],
-                                               floatx16 (&dv)[WANT_DV ? D / 32 : 1], float scale_log2, int q0, int key_row,
-                                               int T, int window, int lane, bool cut = true) {
-  constexpr int KK = D / 16, MT = D / 32;
+// ---- tiles that go from memory into LDS without passing through registers
+// 64 rows of D bf16, unpadded: piece c (16 bytes) of row r in slot c ^ flash_slot(r). The four rows of a transposing read then lie in
+// four different quarters of the banks, and a 16-byte read of 32 rows meets every slot as often as any other.
+template <int D>
+__device__ __forceinline__ constexpr unsigned flash_slot(unsigned r) {
+  return D == 128 ? ((r & 3) << 2 | (r >> 2 & 3)) : ((r >> 1 & 1) << 2 | (r >> 2 & 3));
+}
+typedef __attribute__((address_space(3))) char* LdsBytes;
+__device__ __forceinline__ unsigned lds_address(const void* p) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>((LdsBytes)(p))); }
+__device__ __forceinline__ u32x4 lds_read16(unsigned at) {
+  typedef const u32x4 __attribute__((address_space(3))) * ptr;
+  return *reinterpret_cast<ptr>(static_cast<uintptr_t>(at));
+}
+// A wave's share of a tile's loads: load I moves 1 KiB, WAVES waves take turns.
+template <int D, int WAVES>
+struct TileDma {
+  static constexpr int CPR = D / 8, ROWS = 64 / CPR, LOADS = 64 / (ROWS * WAVES);  // pieces of a row, rows of a load, loads of a wave
+  unsigned first, piece, step;  // bytes: the lane's row, its piece of the row, from load to load
+  unsigned wave;
+  __device__ __forceinline__ TileDma(long rs, int wave_, int lane) : wave(wave_) {
+    const unsigned row = wave_ * ROWS + lane / CPR;
+    first = row * static_cast<unsigned>(rs * 2);
+    piece = (lane % CPR ^ flash_slot<D>(row)) * 16;
+    step = WAVES * ROWS * static_cast<unsigned>(rs * 2);
+  }
+  // The tile that starts at `at`, `rows` of it: what lies past them reads as zeros.
+  __device__ __forceinline__ static u32x4 describe(unsigned long long at, unsigned pitch, int rows) {
+    const int live = min(64, rows);
+    return u32x4{static_cast<unsigned>(at), static_cast<unsigned>(at >> 32) & 0xffffu, live > 0 ? (live - 1) * pitch + D * 2 : 0u, 0x00020000u};
+  }
+  // (Assembly: the compiler would make every LDS read wait for a load into LDS that it knows of.)
+  template <int I>
+  __device__ __forceinline__ void load(const u32x4& rsrc, unsigned tile) const {
+    const unsigned off = first + I * step + (piece ^ flash_slot<D>(I * WAVES * ROWS) * 16);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc),
+                 "s"(tile + (I * WAVES + wave) * 1024)
+                 : "memory");
+  }
+  // The same rows through registers, for planes that are not 16-byte aligned.
+  __device__ __forceinline__ void copy(const unsigned short* first_row, long rs, int rows, char* tile, int lane) const {
+#pragma unroll 1
+    for (int i = 0; i < LOADS; ++i) {
+      const int row = (i * WAVES + static_cast<int>(wave)) * ROWS + lane / CPR, c = lane % CPR;
+      u32x4 x = u32x4{0u, 0u, 0u, 0u};
+      if (row < rows) {
+        const unsigned short* p = first_row + static_cast<long>(row) * rs + c * 8;
+        for (int j = 0; j < 4; ++j) x[j] = p[2 * j] | static_cast<unsigned>(p[2 * j + 1]) << 16;
+      }
+      *reinterpret_cast<u32x4*>(tile + row * (D * 2) + (c ^ flash_slot<D>(row)) * 16) = x;
+    }
+  }
+};
+// Keeps the order of what is written before and after it.
+__device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(4); }  // (but for scalar instructions)
+// A lane's place in a tile: its row as an operand (frag_rows), and its part of the transposing reads (frag_tr).
+template <int D>
+struct TilePlace {
+  unsigned rows, tr;
+  __device__ __forceinline__ explicit TilePlace(int lane) {
+    const unsigned l32 = lane & 31, g = lane >> 5, s = lane & 15, half = lane >> 4 & 1, r = 4 * g + (s >> 2);
+    rows = l32 * (D * 2) + (g ^ flash_slot<D>(l32)) * 16;
+    tr = r * (D * 2) + ((half * 2 + ((s & 3) >> 1)) ^ flash_slot<D>(r)) * 16 + (s & 1) * 8;
+  }
+  __device__ __forceinline__ u32x4 row(unsigned tile, int sub, int kk) const { return lds_read16(((tile + rows) ^ kk * 32) + sub * 64 * D); }
+  __device__ __forceinline__ u32x4 column(unsigned tile, int mt, int sub, int c) const {
+    typedef short4v __attribute__((address_space(3))) * ptr;
+    const unsigned at = tile + tr, imm = (sub * 32 + c * 16) * D * 2;
+    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<ptr>(static_cast<uintptr_t>((at ^ mt * 64) + imm)));
+    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<ptr>(static_cast<uintptr_t>((at ^ mt * 64 ^ 32) + (imm + 8 * D * 2))));
+    const u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
+    return u32x4{a.x, a.y, b.x, b.y};
+  }
+};
+
+// Transposed accumulators of a wave's 32 rows as rows of a [time, D] plane, by way of 32 rows of LDS of the wave's own: whole lines
+// leave the wave where lanes of their own rows would store 8 bytes each.
+template <int D, typename TO>
+__device__ __forceinline__ bool store_acc_rows(TO* __restrict__ plane, long rs, int row0, int time, int lane, const floatx16 (&acc)[D / 32],
+                                               float mul, char* stage) {
+  constexpr int PITCH = D * sizeof(TO), CPR = PITCH / 16, RPI = 64 / CPR;
   const int l32 = lane & 31, lg = lane >> 5;
+  const unsigned slot = flash_slot<128>(l32);
+  bool bad = false;
 #pragma unroll
-  for (int sub = 0; sub < 2; ++sub) {
-    floatx16 sc = zero16(), dp = zero16();
+  for (int mt = 0; mt < D / 32; ++mt)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const float x0 = acc[mt][4 * q4 + 0] * mul, x1 = acc[mt][4 * q4 + 1] * mul, x2 = acc[mt][4 * q4 + 2] * mul,
+                  x3 = acc[mt][4 * q4 + 3] * mul;
+      bad |= !(dev_finite(x0) && dev_finite(x1) && dev_finite(x2) && dev_finite(x3));
+      if constexpr (sizeof(TO) == 2) {
+        *reinterpret_cast<uint2*>(stage + l32 * PITCH + ((mt * 4 + q4) ^ (slot & (CPR - 1))) * 16 + lg * 8) = make_uint2(pack2(x0, x1), pack2(x2, x3));
+      } else {
+        *reinterpret_cast<float4*>(stage + l32 * PITCH + ((mt * 8 + q4 * 2 + lg) ^ slot) * 16) = make_float4(x0, x1, x2, x3);
+      }
+    }
+  bad &= row0 + l32 < time;
+#pragma unroll
+  for (int i = 0; i < 32 / RPI; ++i) {
+    const int r = i * RPI + lane / CPR, c = lane % CPR;
+    const u32x4 x = *reinterpret_cast<const u32x4*>(stage + r * PITCH + (c ^ (flash_slot<128>(r) & (CPR - 1))) * 16);
+    if (row0 + r < time) *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(plane + static_cast<long>(row0 + r) * rs) + c * 16) = x;
+  }
+  return bad;
+}
+
+// The dK/dV pass of one wave over 32 queries x its 32 keys, in three phases whose order the compiler keeps: scores and dP, the
+// transposed operands of the third phase on their way from LDS; P and dS; dV and dK, the next 32 queries on their way.
+// Score accumulators start at -lse / scale and dP at -delta of their rows, so that P = 2^(S scale log2e) and dS / scale = P dP. At
+// head_dim 128 they are read as such, a row's value by every lane, with the next rows. At 64 two waves share a SIMD and the 32 registers
+// would not be there: a row's value is 16 bytes, three bf16 parts (all of its 24 bits) and zeros, and comes in by a product with
+// ones (16 x 12 x 1024: 78 us spilling, 73 so; at 128 the two products more per half cost 164 -> 170 us).
+template <int D>
+struct DkvHalf {
+  static constexpr int KK = D / 16, MT = D / 32, TILE = 64 * D * 2, VALUES = 64 * (D == 64 ? 16 : 4);
+  u32x4 q[KK], g[KK], q_start, g_start;  // rows, and what they start at
+  u32x4 gt[2][MT], qt[2][MT];
+  floatx16 sc, dp;
+  u32x4 pb[2], dsb[2];
+  // Rows `sub` of the set at `set`, piece kk, and their values.
+  __device__ __forceinline__ void fetch_q(const TilePlace<D>& place, unsigned set, int sub, int kk, int l32, int lg) {
+    q[kk] = place.row(set, sub, kk);
+    fetch_start(q_start, sc, set + 2 * TILE, sub, kk, l32, lg);
+  }
+  __device__ __forceinline__ void fetch_g(const TilePlace<D>& place, unsigned set, int sub, int kk, int l32, int lg) {
+    g[kk] = place.row(set + TILE, sub, kk);
+    fetch_start(g_start, dp, set + 2 * TILE + VALUES, sub, kk, l32, lg);
+  }
+  __device__ __forceinline__ static void fetch_start(u32x4& parts, floatx16& acc, unsigned at, int sub, int kk, int l32, int lg) {
+    if constexpr (D == 64) {
+      if (kk == 0) parts = lds_read16(at + l32 * 16 + sub * 512);
+    } else if (kk < 4) {
+      const u32x4 x = lds_read16(at + lg * 16 + (sub * 32 + 8 * kk) * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[4 * kk + j] = __uint_as_float(x[j]);
+    }
+  }
+  __device__ __forceinline__ void fetch(const TilePlace<D>& place, unsigned set, int sub, int l32, int lg) {
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      sc = mfma(frag_rows<D>(q_rows, sub, kk, l32, lg), kf[kk], sc);
-      if constexpr (WANT_DK) dp = mfma(frag_rows<D>(g_rows, sub, kk, l32, lg), vf[kk], dp);
+      fetch_q(place, set, sub, kk, l32, lg);
+      fetch_g(place, set, sub, kk, l32, lg);
     }
-    if (GENERAL == 1 || (GENERAL == 2 && cut)) {
+  }
+  // Row `row`'s value x into a set.
+  __device__ __forceinline__ static void store_value(char* at, int row, float x) {
+    if constexpr (D == 64) {
+      const unsigned hi = pack2(x, 0.0f);
+      const float r1 = x - __uint_as_float(hi << 16);
+      const unsigned mid = pack2(r1, 0.0f);
+      const float r2 = r1 - __uint_as_float(mid << 16);
+      *reinterpret_cast<u32x4*>(at + row * 16) = u32x4{hi | mid << 16, pack2(r2, 0.0f), 0u, 0u};
+    } else {
+      *reinterpret_cast<float*>(at + row * 4) = x;
+    }
+  }
+  __device__ __forceinline__ void scores(const u32x4 (&kf)[KK], const u32x4 (&vf)[KK], const u32x4& ones, const TilePlace<D>& place, unsigned set,
+                                         int sub) {
+    if constexpr (D == 64) {
+      sc = mfma(q_start, ones, zero16());
+      pin();
+      dp = mfma(g_start, ones, zero16());
+      pin();
+    }
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      sc = mfma(q[kk], kf[kk], sc);
+      gt[kk / MT][kk % MT] = place.column(set + TILE, kk % MT, sub, kk / MT);
+      pin();
+      dp = mfma(g[kk], vf[kk], dp);
+      qt[kk / MT][kk % MT] = place.column(set, kk % MT, sub, kk / MT);
+      pin();
+    }
+  }
+  __device__ __forceinline__ void weights(bool cut, float scale_log2, int q0, int key_row, int T, int window, int lg) {
+    if (__builtin_expect(cut, 0)) {
+      asm volatile("");  // (a branch: as selects, the test would go with every tile)
 #pragma unroll
       for (int vv = 0; vv < 16; ++vv) {
-        const int qi = q0 + sub * 32 + acc_row(vv, lg);
+        const int qi = q0 + acc_row(vv, lg);
         const bool masked = key_row > qi || qi >= T || key_row >= T || (window > 0 && key_row + window <= qi);
         sc[vv] = masked ? -INFINITY : sc[vv];
       }
     }
-    // P = 2^(s * scale * log2e - lse * log2e); dS / scale = P (dP - delta): the scale joins dK at the end.
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const float4 l4 = *reinterpret_cast<const float4*>(lse_s + sub * 32 + 8 * q4 + 4 * lg);
-      const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
-      float dl[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if constexpr (WANT_DK) {
-        const float4 d4 = *reinterpret_cast<const float4*>(del_s + sub * 32 + 8 * q4 + 4 * lg);
-        dl[0] = d4.x;
-        dl[1] = d4.y;
-        dl[2] = d4.z;
-        dl[3] = d4.w;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int vv = 4 * q4 + j;
-        const float p = __builtin_amdgcn_exp2f(fmaf(sc[vv], scale_log2, -lv[j]));
-        if constexpr (WANT_DK) dp[vv] = p * (dp[vv] - dl[j]);
-        sc[vv] = p;
-      }
+    for (int vv = 0; vv < 16; ++vv) {
+      const float p = __builtin_amdgcn_exp2f(sc[vv] * scale_log2);
+      dp[vv] *= p;
+      sc[vv] = p;
     }
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      u32x4 pb = u32x4{0u, 0u, 0u, 0u}, dsb = u32x4{0u, 0u, 0u, 0u};
-      if constexpr (WANT_DV) pb = pack8(sc, c);
-      if constexpr (WANT_DK) dsb = pack8(dp, c);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (WANT_DV) dv[mt] = mfma(frag_tr<D>(g_rows, mt, sub, c, lane), pb, dv[mt]);
-        if constexpr (WANT_DK) dk[mt] = mfma(frag_tr<D>(q_rows, mt, sub, c, lane), dsb, dk[mt]);
-      }
+      pb[c] = pack8(sc, c);
+      dsb[c] = pack8(dp, c);
     }
+    pin();
   }
-}
+  // `between(i)`, i of KK, after each pair of products.
+  template <typename F>
+  __device__ __forceinline__ void sums(floatx16 (&dk)[MT], floatx16 (&dv)[MT], const TilePlace<D>& place, unsigned next, int next_sub, int l32, int lg,
+                                       F between) {
+    for_sequence<KK>([&](auto i) {
+      constexpr int kk = decltype(i)::value, c = kk / MT, mt = kk % MT;
+      dv[mt] = mfma(gt[c][mt], pb[c], dv[mt]);
+      fetch_q(place, next, next_sub, kk, l32, lg);
+      pin();
+      dk[mt] = mfma(qt[c][mt], dsb[c], dk[mt]);
+      fetch_g(place, next, next_sub, kk, l32, lg);
+      between(i);
+      pin();
+    });
+  }
+};
 
-// One key block of one KV head: the loop over the query tiles that see it, accumulating dK
-// (WANT_DK) and / or dV (WANT_DV) for the wave's 32 keys, then their stores. head_dim 64 runs it
-// once for both. At head_dim 128 the two accumulator sets (128 registers), both key / value
-// fragments (64) and the score tiles do not fit the 256 registers of two waves per SIMD, so the
-// block is walked twice, once per gradient; the second walk recomputes the scores.
+// One key block of one KV head: the loop over the query tiles that see it, accumulating dK and dV for the wave's 32 keys, then their
+// stores. head_dim 64: two waves per SIMD; at 128 the two sums (128 registers), keys and values (64) and the operands on their way
+// take more than 256 registers, so one wave has its SIMD to itself, and everything it waits for has to be on its way: tiles go straight
+// into LDS a tile ahead, operands come from LDS a phase ahead (DkvHalf), rows go out whole lines at a time.
+// What bounds it: products and vector work, which do not overlap, about 0.6 of the time; then the first tile and the last rows (5 us a
+// workgroup at 128). us, through registers (two walks at 128, scores formed twice) / now: 4 x 16 x 2048 x 128: 220 / 159; 8 x 16 x 1024 x
+// 128: 143 / 106; 16 x 12 x 1024 x 64: 85 / 70; 8 x 12 x 1024 x 64: 47 / 41. Waiting for a tile, storing it and asking for the next were
+// 1500 of 5900 clocks a tile, the waits for operands 1000.
 // GROUPS > 1: groups of the waves take the query tiles of 128 / GROUPS keys in turn, as in the forward.
 // SPLIT: the tiles of s.kv_parts workgroups are consecutive shares of the sequence over the heads, this one's is `part`, and its sums go
 // out as rows of gk and gv, each [part][b, KV head][time][D].
-template <int D, typename TO, bool WANT_DK, bool WANT_DV, bool WIN, int GROUPS, bool SPLIT>
+template <int D, typename TO, int GROUPS, bool SPLIT>
 __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict__ q,
                                                 const unsigned short* __restrict__ k,
                                                 const unsigned short* __restrict__ v, const float* __restrict__ lse,
                                                 const float* __restrict__ delta, const unsigned short* __restrict__ gy,
                                                 TO* __restrict__ gk, TO* __restrict__ gv, const FlashShape& s, char* lds,
                                                 int kb, int b, int gidx, int part) {
-  constexpr int NT = FT / GROUPS, ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;
-  constexpr int KK = D / 16, MT = D / 32, NL = 8 * D / NT;
-  constexpr int SET = flash_dkv_set(D);
-  const int lane = threadIdx.x & 63, l32 = lane & 31, lg = lane >> 5, tid = threadIdx.x % NT;
+  constexpr int ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;
+  constexpr int KK = D / 16, MT = D / 32, TILE = 64 * D * 2, SET = flash_dkv_set(D);
+  typedef TileDma<D, ROW_WAVES> Dma;
+  const int lane = threadIdx.x & 63, l32 = lane & 31, lg = lane >> 5;
   const int group = GROUPS == 1 ? 0 : wave_index() / ROW_WAVES, wave = GROUPS == 1 ? wave_index() : wave_index() % ROW_WAVES;
   char* const smem = lds + group * (2 * SET);
+  const unsigned sets = lds_address(smem);
   const int T = s.time;
-  const TileFetch<D, NT> fetch_q(s.q.rs, T), fetch_g(s.o.rs, T);
+  const Dma dma_q(s.q.rs, wave, lane), dma_g(s.o.rs, wave, lane);
+  const TilePlace<D> place(lane);
   const long kv_off = b * s.kv.bs + gidx * s.kv.hs;
   const int wave_k0 = kb * ROWS + wave * 32;
   const int key_row = wave_k0 + l32;
-  u32x4 kf[KK], vf[WANT_DK ? KK : 1];
-  row_frags<D>(k + kv_off, s.kv.rs, key_row, T, lg, kf);
-  if constexpr (WANT_DK) row_frags<D>(v + kv_off, s.kv.rs, key_row, T, lg, vf);
-  floatx16 dk[WANT_DK ? MT : 1], dv[WANT_DV ? MT : 1];
-#pragma unroll
-  for (int mt = 0; mt < (WANT_DK ? MT : 1); ++mt) dk[mt] = zero16();
-#pragma unroll
-  for (int mt = 0; mt < (WANT_DV ? MT : 1); ++mt) dv[mt] = zero16();
-  const float scale_log2 = s.scale * LOG2E;
   const int block_k0 = kb * ROWS, block_k1 = min(T - 1, kb * ROWS + ROWS - 1);
   const int qt_first = block_k0 / 64;
   const int qt_last = (s.window > 0 ? min(T - 1, block_k1 + s.window - 1) : T - 1) / 64;
-  bool bad = false;
-  // One flat sequence of (query head of the group, query tile), ascending, so the
-  // next tile's global loads can be in flight while the current one is multiplied.
+  // One flat sequence of (query head of the group, query tile), ascending, so that the next tiles can be on their way.
   const int nq = qt_last - qt_first + 1;
   // The workgroup's tiles (none of a late key block's may be left for a late part: its sums are zeros then).
   const int share_at = SPLIT ? static_cast<int>(static_cast<long>(s.rep) * nq * part / s.kv_parts) : 0;
   const int share = (SPLIT ? static_cast<int>(static_cast<long>(s.rep) * nq * (part + 1) / s.kv_parts) : s.rep * nq) - share_at;
   const int r_first = SPLIT ? share_at / nq : 0, qt_start = SPLIT ? qt_first + share_at % nq : qt_first;
   const int steps = (share - group + GROUPS - 1) / GROUPS;  // this group's: GROUPS tiles apart
-  u32x4 rq[NL], rg[NL];
-  float row_lse = 0.0f, row_del = 0.0f;
-  // (head of the group, query tile) of the tile being fetched.
-  int fetch_r = r_first, fetch_qt = qt_start;
-  auto skip = [&](int& r, int& qt, int tiles) {
+  // The tile that is loaded next: its head of the group, what is left of that, and where it lies.
+  const unsigned pitch_q = static_cast<unsigned>(s.q.rs * 2), pitch_g = static_cast<unsigned>(s.o.rs * 2);
+  int next_r = r_first, next_qt = qt_start;
+  const unsigned short *next_q, *next_g;
+  long next_row;
+  auto head = [&]() {
+    const long h = static_cast<long>(gidx) * s.rep + min(next_r, s.rep - 1);  // (past the last tile nothing is loaded)
+    next_q = q + b * s.q.bs + h * s.q.hs + static_cast<long>(next_qt) * 64 * s.q.rs;
+    next_g = gy + b * s.o.bs + h * s.o.hs + static_cast<long>(next_qt) * 64 * s.o.rs;
+    next_row = (static_cast<long>(b) * s.heads + h) * T + next_qt * 64;
+  };
+  auto skip = [&]() {
+    next_q += 64 * s.q.rs;
+    next_g += 64 * s.o.rs;
+    next_row += 64;
+    if (++next_qt > qt_last) {
+      next_qt = qt_first;
+      ++next_r;
+      head();
+    }
+  };
+  head();
+  for (int i = 0; i < group; ++i) skip();
+  // The tile on its way: a lane's row value, two loads a wave where it is the group's only one.
+  constexpr int VALUES = ROW_WAVES > 1 ? 1 : 2;
+  const int value_of = wave & 1;  // 0: lse, 1: delta (other waves repeat them)
+  const unsigned short *coming_q = next_q, *coming_g = next_g;
+  int coming_q0 = 0;
+  float value[VALUES];
+  u32x4 rsrc_q, rsrc_g;
+  auto aim = [&](bool more) {  // (past the last tile: zeros)
+    coming_q = next_q;
+    coming_g = next_g;
+    coming_q0 = next_qt * 64;
+    rsrc_q = Dma::describe(reinterpret_cast<unsigned long long>(next_q), pitch_q, more ? T - coming_q0 : 0);
+    rsrc_g = Dma::describe(reinterpret_cast<unsigned long long>(next_g), pitch_g, more ? T - coming_q0 : 0);
+    const long row = next_row + min(lane, T - 1 - coming_q0);  // (what a row past the end carries is masked)
 #pragma unroll
-    for (int i = 0; i < tiles; ++i)
-      if (++qt > qt_last) {
-        qt = qt_first;
-        ++r;
-      }
+    for (int j = 0; j < VALUES; ++j) value[j] = (VALUES == 2 ? j : value_of) ? delta[row] : lse[row];
+    for (int i = 0; i < GROUPS; ++i) skip();
   };
-  if constexpr (GROUPS > 1) {
-    for (int i = 0; i < group; ++i) skip(fetch_r, fetch_qt, 1);
+  auto load = [&](auto i, unsigned set) {
+    constexpr int I = decltype(i)::value;
+    if constexpr (I < Dma::LOADS) dma_q.template load<I>(rsrc_q, set);
+    else dma_g.template load<I - Dma::LOADS>(rsrc_g, set + TILE);
+  };
+  auto load_all = [&](unsigned set) {
+    for_sequence<2 * Dma::LOADS>([&](auto i) { load(i, set); });
+  };
+  const float start = -1.0f / s.scale;
+  // The set that was on its way is complete for this wave, its rows' values with it.
+  auto arrive = [&](int set) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (__builtin_expect(!s.aligned, 0)) {
+      dma_q.copy(coming_q, s.q.rs, T - coming_q0, smem + set * SET, lane);
+      dma_g.copy(coming_g, s.o.rs, T - coming_q0, smem + set * SET + TILE, lane);
+    }
+#pragma unroll
+    for (int j = 0; j < VALUES; ++j) {
+      const int which = VALUES == 2 ? j : value_of;
+      DkvHalf<D>::store_value(smem + set * SET + 2 * TILE + which * DkvHalf<D>::VALUES, lane, value[j] * (which ? -1.0f : start));
+    }
+  };
+  auto meet = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    pin();
+  };
+  __syncthreads();  // an earlier block's reads of LDS are done
+  aim(true);
+  load_all(sets);
+  u32x4 kf[KK], vf[KK];
+  row_frags<D>(k + kv_off, s.kv.rs, key_row, T, lg, kf);
+  row_frags<D>(v + kv_off, s.kv.rs, key_row, T, lg, vf);
+  floatx16 dk[MT], dv[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    dk[mt] = zero16();
+    dv[mt] = zero16();
   }
-  auto fetch = [&]() {
-    const int r = GROUPS == 1 && !SPLIT ? fetch_r : min(fetch_r, s.rep - 1), q0 = fetch_qt * 64;
-    skip(fetch_r, fetch_qt, GROUPS);
-    const long q_plane = static_cast<long>(b) * s.heads + static_cast<long>(gidx) * s.rep + r;
-    const long head = static_cast<long>(gidx) * s.rep + r;
-    fetch_q.load(q + b * s.q.bs + head * s.q.hs, q0, rq);
-    fetch_g.load(gy + b * s.o.bs + head * s.o.hs, q0, rg);
-    row_lse = 0.0f;
-    row_del = 0.0f;
-    if (tid < 64 && q0 + tid < T) {
-      row_lse = lse[q_plane * T + q0 + tid];
-      row_del = delta[q_plane * T + q0 + tid];
-      bad |= !(dev_finite(row_lse) && dev_finite(row_del));
-    }
+  const float scale_log2 = s.scale * LOG2E;
+  arrive(0);
+  meet();
+  aim(steps > 1);
+  load_all(sets + SET);
+  // A tile of every wave, one barrier each, between its last weights and its last sums: the next tile is complete by then, and this wave
+  // has read all it needs of this one, whose set the tile after the next goes into.
+  int qt = qt_start;
+  auto turn = [&]() {
+    if (++qt > qt_last) qt = qt_first;
   };
-  auto store_set = [&](char* set) {
-    tile_store_rows<D, NT>(set, rq);
-    tile_store_rows<D, NT>(set + ftile(D), rg);
-    if (tid < 64) {
-      float* stats = reinterpret_cast<float*>(set + 2 * ftile(D));
-      stats[tid] = row_lse * LOG2E;
-      stats[64 + tid] = row_del;
-    }
-  };
-  fetch();
-  __syncthreads();  // an earlier walk's reads of the first set are done
-  store_set(smem);
-  if (steps > 1) fetch();
-  // One step of the tile pipeline, taken by every wave for every tile: wait for set idx, store the
-  // next one into the other set, start the loads of the one after.
-  int idx = 0;
-  const char* q_rows;
-  const char* g_rows;
-  const float* lse_s;
-  const float* del_s;
-  auto advance = [&]() {
-    q_rows = smem + (idx & 1) * SET;
-    g_rows = q_rows + ftile(D);
-    lse_s = reinterpret_cast<const float*>(q_rows + 2 * ftile(D));
-    del_s = lse_s + 64;
-    __syncthreads();  // this set is complete, and every wave is done with the other one
-    if (idx + 1 < steps) {
-      store_set(smem + ((idx & 1) ^ 1) * SET);
-      if (idx + 2 < steps) fetch();
-    }
-    ++idx;
-  };
-  auto tile = [&](auto general, int q0, bool cut = true) {
-    flash_dkv_tile<D, WANT_DK, WANT_DV, decltype(general)::value>(q_rows, g_rows, lse_s, del_s, kf, vf, dk, dv, scale_log2, q0,
-                                                                 key_row, T, s.window, lane, cut);
-  };
-  if constexpr (GROUPS > 1 || SPLIT) {
-    int r = r_first, qt = qt_start;
-    for (int i = 0; i < group; ++i) skip(r, qt, 1);
-    const int rounds = (share + GROUPS - 1) / GROUPS;
-    for (int i = 0; i < rounds; ++i) {
-      advance();
-      const int q0 = qt * 64;
-      if ((SPLIT ? i * GROUPS + group < share : r < s.rep) && wave_k0 < T && q0 + 63 >= wave_k0 && (!WIN || q0 < wave_k0 + 31 + s.window)) {
-        if constexpr (WIN) tile(std::true_type{}, q0);
-        else tile(std::integral_constant<int, 2>{}, q0, q0 < wave_k0 + 32 || q0 + 64 > T || wave_k0 + 31 >= T);
-      }
-      skip(r, qt, GROUPS);
-    }
+  for (int i = 0; i < group; ++i) turn();
+  const u32x4 ones = lg ? u32x4{0u, 0u, 0u, 0u} : u32x4{0x3F803F80u, 0x3F80u, 0u, 0u};
+  const int rounds = (share + GROUPS - 1) / GROUPS;
+  DkvHalf<D> half;
+  half.fetch(place, sets, 0, l32, lg);
+#pragma unroll 1
+  for (int i = 0; i < rounds; ++i) {
+    const unsigned set = sets + (i & 1) * SET, other = sets + ((i & 1) ^ 1) * SET;
+    const int q0 = qt * 64;
+    const bool none = GROUPS > 1 && i * GROUPS + group >= share;  // (this group is through: all of it is masked)
+    const bool cut = none || q0 < wave_k0 + 32 || q0 + 64 > T || wave_k0 + 31 >= T || (s.window > 0 && q0 + 63 >= wave_k0 + s.window);
+    const int from = none ? T : key_row;
+    half.scores(kf, vf, ones, place, set, 0);
+    half.weights(cut, scale_log2, q0, from, T, s.window, lg);
+    half.sums(dk, dv, place, set, 1, l32, lg, [](auto) {});
+    half.scores(kf, vf, ones, place, set, 1);
+    half.weights(cut, scale_log2, q0 + 32, from, T, s.window, lg);
+    arrive((i & 1) ^ 1);
+    meet();
+    aim(i + 2 < steps);
+    pin();
+    half.sums(dk, dv, place, other, 0, l32, lg, [&](auto kk) {
+      constexpr int EACH = 2 * Dma::LOADS / KK;
+      for_sequence<EACH>([&](auto j) { load(std::integral_constant<int, decltype(kk)::value * EACH + decltype(j)::value>{}, set); });
+    });
+    for (int j = 0; j < GROUPS; ++j) turn();
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();  // the last loads into LDS are done
+  bool bad = false;
   if constexpr (GROUPS > 1) {
-    constexpr int PART = ((WANT_DK ? MT : 0) + (WANT_DV ? MT : 0)) * 16 * 64;  // floats of a wave
+    constexpr int PART = 2 * MT * 16 * 64;  // floats of a wave
     float* const meet = reinterpret_cast<float*>(lds);
     __syncthreads();  // every wave is done with the tiles
     if (group > 0) {
@@ -772,67 +968,40 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int vv = 0; vv < 16; ++vv) {
-          if constexpr (WANT_DK) mine[(mt * 16 + vv) * 64] = dk[mt][vv];
-          if constexpr (WANT_DV) mine[((WANT_DK ? MT : 0) * 16 + mt * 16 + vv) * 64] = dv[mt][vv];
+          mine[(mt * 16 + vv) * 64] = dk[mt][vv];
+          mine[(MT * 16 + mt * 16 + vv) * 64] = dv[mt][vv];
         }
     }
     __syncthreads();
-    if (group > 0) return bad;
 #pragma unroll
-    for (int g = 0; g < GROUPS - 1; ++g) {
+    for (int g = 0; g < (group > 0 ? 0 : GROUPS - 1); ++g) {
       const float* part = meet + (g * ROW_WAVES + wave) * PART + lane;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int vv = 0; vv < 16; ++vv) {
-          if constexpr (WANT_DK) dk[mt][vv] += part[(mt * 16 + vv) * 64];
-          if constexpr (WANT_DV) dv[mt][vv] += part[((WANT_DK ? MT : 0) * 16 + mt * 16 + vv) * 64];
+          dk[mt][vv] += part[(mt * 16 + vv) * 64];
+          dv[mt][vv] += part[(MT * 16 + mt * 16 + vv) * 64];
         }
     }
-  }
-  for (int r = 0; GROUPS == 1 && !SPLIT && r < s.rep; ++r) {
-    int qt = qt_first;
-    if constexpr (WIN) {
-      for (; qt <= qt_last; ++qt) {
-        advance();
-        const int q0 = qt * 64;
-        if (q0 + 63 >= wave_k0 && q0 < wave_k0 + 31 + s.window) tile(std::true_type{}, q0);
-      }
-    } else if (wave_k0 < T) {  // (a wave whose keys all lie past the sequence end only keeps the barriers)
-      // The wave's first key is a multiple of 32 and a tile's first query a multiple of 64, so the
-      // diagonal cuts one tile, the first the wave takes. The tiles after it need no mask until the
-      // sequence ends inside one, or inside the wave's keys; their loop holds nothing else.
-      const int diag_qt = wave_k0 / 64;
-      for (; qt < diag_qt; ++qt) advance();  // tiles of the block's earlier waves
-      advance();
-      tile(std::true_type{}, qt * 64);
-      ++qt;
-      const int plain_last = wave_k0 + 31 >= T ? qt - 1 : (T / 64) - 1;  // the last tile that ends inside the sequence
-      for (; qt <= min(plain_last, qt_last); ++qt) {
-        advance();
-        tile(std::false_type{}, qt * 64);
-      }
-      for (; qt <= qt_last; ++qt) {
-        advance();
-        tile(std::true_type{}, qt * 64);
-      }
-    }
-    for (; qt <= qt_last; ++qt) advance();
+    __syncthreads();  // (read before the rows go out through the same memory)
+    if (group > 0) return bad;
   }
   const long out_off = SPLIT ? ((static_cast<long>(part) * s.batch + b) * s.kv_heads + gidx) * T * D : kv_off, out_rs = SPLIT ? D : s.kv.rs;
-  if constexpr (WANT_DK) bad |= store_transposed_acc<D, TO>(gk + out_off, out_rs, key_row, T, lg, dk, s.scale);
-  if constexpr (WANT_DV) bad |= store_transposed_acc<D, TO>(gv + out_off, out_rs, key_row, T, lg, dv, 1.0f);
+  char* const stage = lds + wave * (32 * D * static_cast<int>(sizeof(TO)));
+  bad |= store_acc_rows<D, TO>(gk + out_off, out_rs, wave_k0, T, lane, dk, s.scale, stage);
+  bad |= store_acc_rows<D, TO>(gv + out_off, out_rs, wave_k0, T, lane, dv, 1.0f, stage);
   return bad;
 }
 
-template <int D, typename TO, bool WIN, int GROUPS, bool SPLIT>
+template <int D, typename TO, int GROUPS, bool SPLIT>
 __global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_dkv_kernel(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const float* __restrict__ lse, const float* __restrict__ delta, const unsigned short* __restrict__ gy,
     TO* __restrict__ gk, TO* __restrict__ gv, FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
   // Two sets of (query tile, gradient tile, 64 log-sum-exp values, 64 row terms): the next set is
   // stored while this one is multiplied, so a tile costs one barrier.
-  __shared__ __attribute__((aligned(16))) char smem[GROUPS * 2 * flash_dkv_set(D)];
+  __shared__ __attribute__((aligned(256))) char smem[GROUPS * 2 * flash_dkv_set(D)];
   // Early key blocks are seen by the most queries: a workgroup takes one of them and then its
   // mirror image from the back (see the forward kernel).
   const int k_blocks = (s.time + 128 / GROUPS - 1) / (128 / GROUPS);
@@ -849,17 +1018,12 @@ __global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_dkv_
   } else {
     flash_block_of((k_blocks + 1) / 2, s.batch * s.kv_heads, &pair, &kv_plane);
   }
-  const int gidx = static_cast<int>(kv_plane % s.kv_heads), b = static_cast<int>(kv_plane / s.kv_heads);
+  const int b = static_cast<int>(kv_plane) / s.kv_heads, gidx = static_cast<int>(kv_plane) - b * s.kv_heads;
   bool bad = false;
   for (int pass = 0; pass < (SPLIT || s.kv_single ? 1 : 2); ++pass) {
     const int kb = pass == 0 ? pair : k_blocks - 1 - pair;
     if (pass == 1 && kb <= pair) break;
-    if constexpr (D == 64) {
-      bad |= flash_dkv_block<D, TO, true, true, WIN, GROUPS, SPLIT>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx, part);
-    } else {
-      bad |= flash_dkv_block<D, TO, false, true, WIN, GROUPS, SPLIT>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx, part);
-      bad |= flash_dkv_block<D, TO, true, false, WIN, GROUPS, SPLIT>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx, part);
-    }
+    bad |= flash_dkv_block<D, TO, GROUPS, SPLIT>(q, k, v, lse, delta, gy, gk, gv, s, smem, kb, b, gidx, part);
   }
   if (bad) dev_raise_fault(fault, tag);
 }
@@ -1177,6 +1341,7 @@ FlashShape make_shape(uint64_t batch, uint64_t heads, uint64_t kv_heads, uint64_
   s.rep = static_cast<int>(heads / kv_heads);
   s.q_single = s.kv_single = 0;
   s.kv_parts = 1;
+  s.aligned = 0;
   s.scale = scale;
   return s;
 }
@@ -1268,30 +1433,36 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
   for_groups<D>(groups, with_groups);
 }
 
-// Into how many parts the query tiles that a key block sees are split (1: none), and the groups of waves that go with it. The pass has a
-// workgroup per key block and KV head, so few KV heads leave units idle however many query heads there are, and each workgroup walks
-// the tiles of all of them, 1.9 us apiece. A part is a consecutive share of those tiles on a workgroup of its own; its f32 sums go through
-// scratch to a second launch that adds them in order. The estimate is the root of the squares of the longest walk and of the
-// chip's work, per key block of 128 or 64 keys, fitted to 24 shapes x 3 group counts x 9 part counts; the second launch takes 4.5 us
-// or 0.13 us a megabyte. Taken where that is an eighth less, for the fit is no better (15 to 25 %).
-// us of the pass, before / now: 10 x 13 heads over one x 670: 112 / 47; 5 x 2 over 1 x 1161 x 128, window 612: 92 / 45;
-// 8 over 2 x 291 x 128: 77 / 24; 2 x 8 over 2 x 1024 x 128: 186 / 47; 15 x 14 over 2 x 122: 26 / 19; 5 x 1000 x 128: 58 / 34;
-// 4 x 4096: 56 / 44. Many planes (8 x 12 x 1024: 49, split in two 77) stay as they are.
-int flash_kv_parts(omx_ctx* ctx, const FlashShape& s, int dim, int* groups) {
-  if (ctx->flash_kv_parts) return ctx->flash_kv_parts;
-  if (ctx->flash_schedule != 0) return 1;
+// How the key side's pass is cut: groups of waves that take a key block's query tiles in turn, and parts, consecutive shares of those
+// tiles on workgroups of their own, whose f32 sums go through scratch to a second launch that adds them in order. The pass has a
+// workgroup per key block and KV head, so few KV heads leave units idle however many query heads there are, and a workgroup walks the
+// tiles of all of them, 1.3 to 1.7 us apiece. The estimate is the root of the squares of the longest walk and of the chip's work, per
+// key block of 128, 64 or 32 keys, fitted to 24 shapes x 3 group counts x 8 part counts (rms 6 to 12 %); the second launch takes 4.5 us
+// or 2 us and 0.14 us a megabyte. Parts are taken where they gain a twentieth. Over those shapes the choice takes 2.5 % more than the
+// best of all counts on average, 12 % at most. us of the pass, one group and part / by the rule: 10 x 13 heads over one x 670: 201 /
+// 43; 2 x 8 over 2 x 1024 x 128: 114 / 35; 8 over 2 x 291 x 128: 51 / 27; 12 x 2048: 42 / 31; 8 x 1024: 24 / 15; many planes (8 x 12
+// x 1024: 44) stay whole.
+struct FlashKeyPlan {
+  int groups, parts, whole_groups;  // whole_groups: without parts
+};
+FlashKeyPlan flash_key_plan(omx_ctx* ctx, const FlashShape& s, int dim) {
   const long units = ctx->cu_count > 0 ? ctx->cu_count : 256, planes = static_cast<long>(s.batch) * s.kv_heads;
-  if (planes * ((s.time + 127) / 128) >= 2 * units) return 1;
+  if (ctx->flash_schedule != 0) {  // forced (tests)
+    const int groups = ctx->flash_schedule < 3 ? 1 : std::min(dim == 64 ? 4 : 2, ctx->flash_schedule == 3 ? 2 : 4);
+    return {groups, std::max(1, ctx->flash_kv_parts), groups};
+  }
+  if (planes * ((s.time + 127) / 128) >= 2 * units) return {1, std::max(1, ctx->flash_kv_parts), 1};
   struct Fit {
     double first, step, work, each;  // us: of a workgroup, of a tile on its way; of a unit's tiles, of a unit's workgroups
   };
-  const Fit fits[2][2] = {{{7.6, 1.9, 0.74, 4.07}, {7.66, 2.08, 0.78, 3.5}}, {{12.23, 4.74, 0.77, 10.93}, {11.53, 5.68, 2.84, 12.98}}};
+  const Fit fits[2][3] = {{{10.1, 1.27, 0.59, 4.03}, {10.4, 1.36, 0.86, 4.05}, {9.7, 1.72, 1.61, 8.17}},
+                          {{13.2, 1.53, 1.45, 9.4}, {15.2, 1.54, 1.50, 10.9}, {}}};
   const double megabytes = 8e-6 * static_cast<double>(planes) * s.time * dim;
   double whole = 1e30, least = 1e30;
-  int parts = 1, by = 1;
-  for (int g = 1; g <= 2; ++g) {
-    const Fit& f = fits[dim == 128][g - 1];
-    const int rows = 128 / g, blocks = (s.time + rows - 1) / rows;
+  FlashKeyPlan plan = {1, 1, 1};
+  for (int shift = 0; shift < (dim == 64 ? 3 : 2); ++shift) {
+    const int g = 1 << shift, rows = 128 / g, blocks = (s.time + rows - 1) / rows;
+    const Fit& f = fits[dim == 128][shift];
     long all = 0, most = 0;
     for (int kb = 0; kb < blocks; ++kb) {
       const int last = s.window > 0 ? std::min<long>(s.time - 1, std::min(s.time - 1, kb * rows + rows - 1) + static_cast<long>(s.window) - 1) : s.time - 1;
@@ -1300,23 +1471,25 @@ int flash_kv_parts(omx_ctx* ctx, const FlashShape& s, int dim, int* groups) {
       most = std::max(most, tiles);
     }
     for (const int p : {1, 2, 3, 4, 6, 8, 12, 16, 24}) {
-      if (p > most || (p > 1 && p * megabytes > 256.0)) break;
+      if (p > 1 && (p > most || p * megabytes > 256.0)) break;
       const double groups_of_units = static_cast<double>(blocks * planes * p) / static_cast<double>(units);
       const double walk = f.first + f.step * static_cast<double>((most + p * g - 1) / (p * g));
       const double work = f.work * (static_cast<double>(all * planes) / static_cast<double>(g * units) + (p * g > 1 ? 0.5 * groups_of_units : 0.0)) + f.each * groups_of_units;
-      const double us = std::sqrt(walk * walk + work * work) + (p > 1 ? std::max(4.5, 2.5 + 0.13 * megabytes * p) : 0.0);
-      if (p == 1) {
-        whole = std::min(whole, us);
-      } else if (us < least) {
+      const double us = std::sqrt(walk * walk + work * work) + (p > 1 ? std::max(4.5, 2.0 + 0.14 * megabytes * p) : 0.0);
+      if (p == 1 && us < whole) {
+        whole = us;
+        plan.whole_groups = g;
+      }
+      if (p > 1 && us < least) {
         least = us;
-        parts = p;
-        by = g;
+        plan.groups = g;
+        plan.parts = p;
       }
     }
   }
-  if (least >= 0.875 * whole) return 1;
-  *groups = by;
-  return parts;
+  if (least >= 0.95 * whole) plan = {plan.whole_groups, 1, plan.whole_groups};
+  if (ctx->flash_kv_parts) plan = {plan.whole_groups, ctx->flash_kv_parts, plan.whole_groups};
+  return plan;
 }
 
 template <int D>
@@ -1333,14 +1506,13 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
   const unsigned kv_planes = static_cast<unsigned>(s.batch * s.kv_heads), q_planes = static_cast<unsigned>(s.batch * s.heads);
   const int tiles = flash_tiles(s);
   const int q_groups = flash_groups(ctx, q_planes, s.time, tiles, s.window > 0, D);
-  int kv_groups = flash_groups(ctx, kv_planes, s.time, static_cast<int>(std::min<long>(static_cast<long>(tiles) * s.rep, 1 << 20)), s.window > 0, D);
+  const FlashKeyPlan plan = flash_key_plan(ctx, s, D);
   // Split where that takes less and there is room for the sums, in as many parts as there is room for.
   const long kv_total = static_cast<long>(kv_planes) * s.time * D;
   float* parts = nullptr;
-  int split_groups = kv_groups;
-  for (s.kv_parts = flash_kv_parts(ctx, s, D, &split_groups); s.kv_parts > 1; --s.kv_parts)
+  for (s.kv_parts = plan.parts; s.kv_parts > 1; --s.kv_parts)
     if ((parts = static_cast<float*>(omx_workspace_if_room(ctx, static_cast<uint64_t>(s.kv_parts) * kv_total * 8, kExtraSlot)))) break;
-  if (s.kv_parts > 1) kv_groups = split_groups;
+  const int kv_groups = s.kv_parts > 1 ? plan.groups : plan.whole_groups;
   const unsigned q_rows = 128 / q_groups, kv_rows = 128 / kv_groups;
   s.q_single = q_groups > 1 || flash_single(ctx, pairs * q_planes, D == 64 ? 3 : 2, false);
   s.kv_single = kv_groups > 1 || flash_single(ctx, pairs * kv_planes, 2, true);
@@ -1364,10 +1536,8 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
     for_groups<D>(kv_groups, [&](auto count) {
       constexpr int G = decltype(count)::value;
       float* const part_v = parts + s.kv_parts * kv_total;
-      if (s.kv_parts > 1 && s.window > 0) go_dkv(flash_bwd_dkv_kernel<D, float, true, G, true>, parts, part_v);
-      else if (s.kv_parts > 1) go_dkv(flash_bwd_dkv_kernel<D, float, false, G, true>, parts, part_v);
-      else if (s.window > 0) go_dkv(flash_bwd_dkv_kernel<D, T, true, G, false>, gk_ptr, gv_ptr);
-      else go_dkv(flash_bwd_dkv_kernel<D, T, false, G, false>, gk_ptr, gv_ptr);
+      if (s.kv_parts > 1) go_dkv(flash_bwd_dkv_kernel<D, float, G, true>, parts, part_v);
+      else go_dkv(flash_bwd_dkv_kernel<D, T, G, false>, gk_ptr, gv_ptr);
     });
     if (s.kv_parts > 1)
       omx_launch_timed(ctx, flash_parts_kernel<D, T>, dim3(static_cast<unsigned>((kv_total / 8 + 255) / 256), 2), dim3(256), 0, nullptr,
@@ -1421,6 +1591,8 @@ int32_t omx_flash_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, cons
                     (unsigned long long)dim);
   FlashShape s = make_shape(batch, heads, kv_heads, time, dim, window, scale, strides);
   if (int32_t rc = check_row_strides(ctx, s); rc != OMX_OK) return rc;
+  s.aligned = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(gy)) & 15u) == 0 &&
+              ((s.q.rs | s.q.hs | s.q.bs | s.kv.rs | s.kv.hs | s.kv.bs | s.o.rs | s.o.hs | s.o.bs) & 7) == 0;
   const long rows = static_cast<long>(batch * heads * time);
   void* ws = nullptr;
   int32_t rc = omx_workspace(ctx, rows * sizeof(float), &ws);

@@ -1030,6 +1030,29 @@ def test_causal_sdpa_bf16_with_a_key_block_s_tiles_shared_by_workgroups(be, shap
         be.set_option("flash_kv_parts", 0)
 
 
+@pytest.mark.parametrize("groups", [1, 2, 4])
+@pytest.mark.parametrize("shape,hkv,window", [((1, 2, 97, 64), 1, None), ((1, 2, 130, 128), 2, 70), ((1, 4, 200, 64), 2, 33)])
+def test_causal_sdpa_bf16_backward_of_rows_that_are_not_16_byte_aligned(be, shape, hkv, window, groups):
+    """Tiles go straight into LDS only from 16-byte rows; others are copied there, and every bit of the gradients is the same."""
+    from ojas_amd.backend import BF16, DeviceTensor
+
+    b, h, t, d = shape
+    rng = np.random.default_rng(t)
+    x = [rng.normal(size=(b, n, t, d)).astype(np.float32) for n in (h, hkv, hkv, h)]
+    aligned = [be.upload(a, BF16) for a in x]
+    wider = [be.upload(np.concatenate([np.zeros(2, np.float32), a.ravel()]), BF16) for a in x]
+    shifted = [DeviceTensor(be, w.ptr + 4, a.shape, BF16, owns=False) for w, a in zip(wider, x)]
+    be.set_option("flash_schedule", {1: 1, 2: 3, 4: 4}[groups])
+    try:
+        out, lse = be.causal_sdpa_forward(*aligned[:3], window, out_dtype=BF16)
+        want = be.causal_sdpa_backward(*aligned[:3], out, lse, aligned[3], window, grad_dtype=BF16)
+        got = be.causal_sdpa_backward(*shifted[:3], out, lse, shifted[3], window, grad_dtype=BF16)
+        for a, e in zip(got, want):
+            np.testing.assert_array_equal(be.download_f32(a), be.download_f32(e))
+    finally:
+        be.set_option("flash_schedule", 0)
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("shared", [(0, 4, 0), (0, 0, 4), (4, 4, 4)])
 def test_causal_attention_keeps_its_accuracy_when_rows_share_a_component(be, dim, shared):
