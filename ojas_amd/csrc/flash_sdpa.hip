@@ -40,7 +40,7 @@ constexpr int fpitch(int D) { return D * 2 + 16; }      // bytes per LDS row: D 
 constexpr int ftile(int D) { return 64 * fpitch(D); }   // a 64-row tile
 constexpr int FT = 256;                                 // threads per block (4 waves of 32 rows)
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr int flash_dkv_set(int D) { return 2 * 64 * D * 2 + 2 * 64 * (D == 64 ? 16 : 4); }  // bytes: query and gradient tile, two values a row (DkvHalf)
+constexpr int flash_dkv_set(int D) { return 2 * 64 * D * 2 + 2 * 64 * 4; }  // bytes: query and gradient tile, two values a row
 constexpr int flash_dkv_waves(int D, int groups) { return D == 64 && groups <= 2 ? 2 : 1; }
 // Waves per SIMD the query-side passes are compiled for: what their LDS leaves room for.
 constexpr int flash_waves(int D, int groups) { return groups == 1 ? (D == 64 ? 3 : 2) : groups == 2 && D == 64 ? 2 : 1; }
@@ -689,69 +689,48 @@ __device__ __forceinline__ bool store_acc_rows(TO* __restrict__ plane, long rs, 
 
 // The dK/dV pass of one wave over 32 queries x its 32 keys, in three phases whose order the compiler keeps: scores and dP, the
 // transposed operands of the third phase on their way from LDS; P and dS; dV and dK, the next 32 queries on their way.
-// Score accumulators start at -lse / scale and dP at -delta of their rows, so that P = 2^(S scale log2e) and dS / scale = P dP. At
-// head_dim 128 they are read as such, a row's value by every lane, with the next rows. At 64 two waves share a SIMD and the 32 registers
-// would not be there: a row's value is 16 bytes, three bf16 parts (all of its 24 bits) and zeros, and comes in by a product with
-// ones (16 x 12 x 1024: 78 us spilling, 73 so; at 128 the two products more per half cost 164 -> 170 us).
+// The rows' values, log-sum-exp (times log2 e) and delta, are read by every lane for its accumulator's rows: at head_dim 128 with the
+// next rows, at 64, where two waves share a SIMD, with the transposed operands.
 template <int D>
 struct DkvHalf {
-  static constexpr int KK = D / 16, MT = D / 32, TILE = 64 * D * 2, VALUES = 64 * (D == 64 ? 16 : 4);
-  u32x4 q[KK], g[KK], q_start, g_start;  // rows, and what they start at
+  static constexpr int KK = D / 16, MT = D / 32, TILE = 64 * D * 2;
+  static constexpr bool EARLY = D == 128;
+  u32x4 q[KK], g[KK];  // rows
   u32x4 gt[2][MT], qt[2][MT];
+  float4 lse[4], del[4];
   floatx16 sc, dp;
   u32x4 pb[2], dsb[2];
-  // Rows `sub` of the set at `set`, piece kk, and their values.
-  __device__ __forceinline__ void fetch_q(const TilePlace<D>& place, unsigned set, int sub, int kk, int l32, int lg) {
+  // Rows `sub` of the set at `set`, piece kk.
+  __device__ __forceinline__ void fetch_q(const TilePlace<D>& place, unsigned set, int sub, int kk, int lg) {
     q[kk] = place.row(set, sub, kk);
-    fetch_start(q_start, sc, set + 2 * TILE, sub, kk, l32, lg);
+    if (EARLY && kk < 4) lse[kk] = values(set, sub, kk, lg);
   }
-  __device__ __forceinline__ void fetch_g(const TilePlace<D>& place, unsigned set, int sub, int kk, int l32, int lg) {
+  __device__ __forceinline__ void fetch_g(const TilePlace<D>& place, unsigned set, int sub, int kk, int lg) {
     g[kk] = place.row(set + TILE, sub, kk);
-    fetch_start(g_start, dp, set + 2 * TILE + VALUES, sub, kk, l32, lg);
+    if (EARLY && kk < 4) del[kk] = values(set + 256, sub, kk, lg);
   }
-  __device__ __forceinline__ static void fetch_start(u32x4& parts, floatx16& acc, unsigned at, int sub, int kk, int l32, int lg) {
-    if constexpr (D == 64) {
-      if (kk == 0) parts = lds_read16(at + l32 * 16 + sub * 512);
-    } else if (kk < 4) {
-      const u32x4 x = lds_read16(at + lg * 16 + (sub * 32 + 8 * kk) * 4);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[4 * kk + j] = __uint_as_float(x[j]);
-    }
+  __device__ __forceinline__ static float4 values(unsigned set, int sub, int q4, int lg) {
+    return __builtin_bit_cast(float4, lds_read16(set + lg * 16 + (2 * TILE + (sub * 32 + 8 * q4) * 4)));
   }
-  __device__ __forceinline__ void fetch(const TilePlace<D>& place, unsigned set, int sub, int l32, int lg) {
+  __device__ __forceinline__ void fetch(const TilePlace<D>& place, unsigned set, int sub, int lg) {
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      fetch_q(place, set, sub, kk, l32, lg);
-      fetch_g(place, set, sub, kk, l32, lg);
+      fetch_q(place, set, sub, kk, lg);
+      fetch_g(place, set, sub, kk, lg);
     }
   }
-  // Row `row`'s value x into a set.
-  __device__ __forceinline__ static void store_value(char* at, int row, float x) {
-    if constexpr (D == 64) {
-      const unsigned hi = pack2(x, 0.0f);
-      const float r1 = x - __uint_as_float(hi << 16);
-      const unsigned mid = pack2(r1, 0.0f);
-      const float r2 = r1 - __uint_as_float(mid << 16);
-      *reinterpret_cast<u32x4*>(at + row * 16) = u32x4{hi | mid << 16, pack2(r2, 0.0f), 0u, 0u};
-    } else {
-      *reinterpret_cast<float*>(at + row * 4) = x;
-    }
-  }
-  __device__ __forceinline__ void scores(const u32x4 (&kf)[KK], const u32x4 (&vf)[KK], const u32x4& ones, const TilePlace<D>& place, unsigned set,
-                                         int sub) {
-    if constexpr (D == 64) {
-      sc = mfma(q_start, ones, zero16());
-      pin();
-      dp = mfma(g_start, ones, zero16());
-      pin();
-    }
+  __device__ __forceinline__ void scores(const u32x4 (&kf)[KK], const u32x4 (&vf)[KK], const TilePlace<D>& place, unsigned set, int sub, int lg) {
+    sc = zero16();
+    dp = zero16();
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       sc = mfma(q[kk], kf[kk], sc);
       gt[kk / MT][kk % MT] = place.column(set + TILE, kk % MT, sub, kk / MT);
+      if (!EARLY) lse[kk] = values(set, sub, kk, lg);
       pin();
       dp = mfma(g[kk], vf[kk], dp);
       qt[kk / MT][kk % MT] = place.column(set, kk % MT, sub, kk / MT);
+      if (!EARLY) del[kk] = values(set + 256, sub, kk, lg);
       pin();
     }
   }
@@ -765,11 +744,17 @@ struct DkvHalf {
         sc[vv] = masked ? -INFINITY : sc[vv];
       }
     }
+    // P = 2^(s * scale * log2e - lse * log2e); dS / scale = P (dP - delta): the scale joins dK at the end.
 #pragma unroll
-    for (int vv = 0; vv < 16; ++vv) {
-      const float p = __builtin_amdgcn_exp2f(sc[vv] * scale_log2);
-      dp[vv] *= p;
-      sc[vv] = p;
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const float lv[4] = {lse[q4].x, lse[q4].y, lse[q4].z, lse[q4].w}, dl[4] = {del[q4].x, del[q4].y, del[q4].z, del[q4].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int vv = 4 * q4 + j;
+        const float p = __builtin_amdgcn_exp2f(fmaf(sc[vv], scale_log2, -lv[j]));
+        dp[vv] = p * (dp[vv] - dl[j]);
+        sc[vv] = p;
+      }
     }
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
@@ -780,15 +765,15 @@ struct DkvHalf {
   }
   // `between(i)`, i of KK, after each pair of products.
   template <typename F>
-  __device__ __forceinline__ void sums(floatx16 (&dk)[MT], floatx16 (&dv)[MT], const TilePlace<D>& place, unsigned next, int next_sub, int l32, int lg,
+  __device__ __forceinline__ void sums(floatx16 (&dk)[MT], floatx16 (&dv)[MT], const TilePlace<D>& place, unsigned next, int next_sub, int lg,
                                        F between) {
     for_sequence<KK>([&](auto i) {
       constexpr int kk = decltype(i)::value, c = kk / MT, mt = kk % MT;
       dv[mt] = mfma(gt[c][mt], pb[c], dv[mt]);
-      fetch_q(place, next, next_sub, kk, l32, lg);
+      fetch_q(place, next, next_sub, kk, lg);
       pin();
       dk[mt] = mfma(qt[c][mt], dsb[c], dk[mt]);
-      fetch_g(place, next, next_sub, kk, l32, lg);
+      fetch_g(place, next, next_sub, kk, lg);
       between(i);
       pin();
     });
@@ -885,7 +870,6 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
   auto load_all = [&](unsigned set) {
     for_sequence<2 * Dma::LOADS>([&](auto i) { load(i, set); });
   };
-  const float start = -1.0f / s.scale;
   // The set that was on its way is complete for this wave, its rows' values with it.
   auto arrive = [&](int set) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -896,7 +880,7 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
 #pragma unroll
     for (int j = 0; j < VALUES; ++j) {
       const int which = VALUES == 2 ? j : value_of;
-      DkvHalf<D>::store_value(smem + set * SET + 2 * TILE + which * DkvHalf<D>::VALUES, lane, value[j] * (which ? -1.0f : start));
+      *reinterpret_cast<float*>(smem + set * SET + 2 * TILE + which * 256 + lane * 4) = value[j] * (which ? 1.0f : LOG2E);
     }
   };
   auto meet = [&]() {
@@ -929,10 +913,9 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     if (++qt > qt_last) qt = qt_first;
   };
   for (int i = 0; i < group; ++i) turn();
-  const u32x4 ones = lg ? u32x4{0u, 0u, 0u, 0u} : u32x4{0x3F803F80u, 0x3F80u, 0u, 0u};
   const int rounds = (share + GROUPS - 1) / GROUPS;
   DkvHalf<D> half;
-  half.fetch(place, sets, 0, l32, lg);
+  half.fetch(place, sets, 0, lg);
 #pragma unroll 1
   for (int i = 0; i < rounds; ++i) {
     const unsigned set = sets + (i & 1) * SET, other = sets + ((i & 1) ^ 1) * SET;
@@ -940,16 +923,16 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     const bool none = GROUPS > 1 && i * GROUPS + group >= share;  // (this group is through: all of it is masked)
     const bool cut = none || q0 < wave_k0 + 32 || q0 + 64 > T || wave_k0 + 31 >= T || (s.window > 0 && q0 + 63 >= wave_k0 + s.window);
     const int from = none ? T : key_row;
-    half.scores(kf, vf, ones, place, set, 0);
+    half.scores(kf, vf, place, set, 0, lg);
     half.weights(cut, scale_log2, q0, from, T, s.window, lg);
-    half.sums(dk, dv, place, set, 1, l32, lg, [](auto) {});
-    half.scores(kf, vf, ones, place, set, 1);
+    half.sums(dk, dv, place, set, 1, lg, [](auto) {});
+    half.scores(kf, vf, place, set, 1, lg);
     half.weights(cut, scale_log2, q0 + 32, from, T, s.window, lg);
     arrive((i & 1) ^ 1);
     meet();
     aim(i + 2 < steps);
     pin();
-    half.sums(dk, dv, place, other, 0, l32, lg, [&](auto kk) {
+    half.sums(dk, dv, place, other, 0, lg, [&](auto kk) {
       constexpr int EACH = 2 * Dma::LOADS / KK;
       for_sequence<EACH>([&](auto j) { load(std::integral_constant<int, decltype(kk)::value * EACH + decltype(j)::value>{}, set); });
     });
