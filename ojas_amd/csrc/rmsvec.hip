@@ -135,6 +135,62 @@ __global__ __launch_bounds__(RV_THREADS) void rms_fwd_vec_kernel(const TX* __res
   if (bad) dev_raise_fault(fault, tag);
 }
 
+// The same with a workgroup per row, a wave per 256 columns: a lane has one chunk, and a call of few rows, which fetches every
+// instruction and waits once for memory, is a third of the code and a shorter chain (with a launch's 1.4 us in it, us, a wave per row / a
+// workgroup: 1 x 768: 4.4 / 3.2; 64 x 768: 4.6 / 3.2; 1024 x 768: 5.4 / 4.6; 64 x 2048: 8.8 / 4.0; 1024 x 2048: 11.9 / 7.9).
+template <typename TX, typename TA, typename TY>
+__global__ __launch_bounds__(512) void rms_fwd_row_kernel(const TX* __restrict__ x, const TA* __restrict__ add, const float* __restrict__ w,
+                                                          float* __restrict__ sum_out, TY* __restrict__ y, unsigned dim, float eps,
+                                                          OmxFaultWord* fault, unsigned long long tag) {
+  __shared__ float sums[8];
+  const unsigned c = threadIdx.x * 4, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const size_t at = static_cast<size_t>(blockIdx.x) * dim + c;
+  const bool own = c < dim;
+  Raw4<TX> xr;
+  Raw4<TA> ar;
+  Raw4<float> wr;
+  xr.clear();
+  ar.clear();
+  wr.clear();
+  if (own) {
+    xr.load(x + at);
+    if (add) ar.load(add + at);
+    wr.load(w + c);
+  }
+  float xv[4], wv[4], out[4];
+  xr.get(xv);
+  bool bad = false;
+  if (add) {
+    float av[4];
+    ar.get(av);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      xv[e] = xv[e] + av[e];
+      bad |= !dev_finite(xv[e]);
+    }
+    if (own) dev_store4<float>(sum_out, at, xv);
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ss += xv[e] * xv[e];
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) sums[wave] = ss;
+  __syncthreads();
+  ss = sums[0];
+  for (unsigned i = 1; i < waves; ++i) ss += sums[i];
+  const float denom = ss / static_cast<float>(dim) + eps;
+  const float rstd = 1.0f / sqrtf(denom);
+  bad |= !(dev_finite(denom) && denom > 0.0f && dev_finite(rstd));
+  wr.get(wv);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    out[e] = xv[e] * rstd * wv[e];
+    bad |= !dev_finite(out[e]);
+  }
+  if (own) dev_store4<TY>(y, at, out);
+  if (bad) dev_raise_fault(fault, tag);
+}
+
 // A row's sum in every lane for the backward kernel. WIDE rows keep the exchanges through LDS: with wave_sum's swaps and rotations
 // (same order, same bits) the compiler holds fewer of a row's loads at once, 129 registers for 162, at the same three waves per
 // SIMD, and 8192 rows of 2048 took 54.9 us instead of 48.2. Narrow rows gain by wave_sum (figures there).
@@ -331,12 +387,18 @@ int32_t omx_rms_forward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const 
                                                (width(x_dtype) + (add ? width(add_dtype) + 4.0 : 0.0) + width(y_dtype)));
   // Up to half the waves the chip holds (32 per compute unit), nothing else hides a row's latencies.
   const bool together = rows <= 16ull * static_cast<uint64_t>(ctx->cu_count > 0 ? ctx->cu_count : 256);
+  // Three waves of a row and more, up to three quarters of the waves the chip holds (2048 x 768: 6.8 a wave per row, 6.4 a workgroup;
+  // 2730 x 768: 7.9, 8.5). Two waves of a row gain nothing (512 columns, 1 to 1024 rows: within 0.1).
+  const bool by_row = nch >= 3 && rows * nch <= 24ull * static_cast<uint64_t>(ctx->cu_count > 0 ? ctx->cu_count : 256);
 #define RV_FWD(TX, TA, TY, N)                                                                                      \
   omx_launch_timed(ctx, together ? rms_fwd_vec_kernel<TX, TA, TY, N, true> : rms_fwd_vec_kernel<TX, TA, TY, N, false>, grid, block, 0, timer.start(), timer.stop(),            \
                    static_cast<const TX*>(x), static_cast<const TA*>(add), w, sum_out, static_cast<TY*>(y),        \
                    static_cast<size_t>(rows), static_cast<int>(dim), eps, ctx->fault, tag)
 #define RV_FWD_N(TX, TA, TY)      \
-  switch (nch) {                  \
+  if (by_row) \
+    omx_launch_timed(ctx, (rms_fwd_row_kernel<TX, TA, TY>), dim3(static_cast<unsigned>(rows)), dim3(64 * nch), 0, timer.start(), timer.stop(), \
+                   static_cast<const TX*>(x), static_cast<const TA*>(add), w, sum_out, static_cast<TY*>(y), static_cast<unsigned>(dim), eps, ctx->fault, tag); \
+  else switch (nch) {                  \
     case 1: RV_FWD(TX, TA, TY, 1); break; \
     case 2: RV_FWD(TX, TA, TY, 2); break; \
     case 3: RV_FWD(TX, TA, TY, 3); break; \
