@@ -1078,6 +1078,11 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value) {
     ctx->flash_schedule = static_cast<int>(value);
     return OMX_OK;
   }
+  if (name && strcmp(name, "attention_together") == 0) {
+    if (value < -1 || value > 1) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: attention_together takes -1..1");
+    ctx->attention_together = static_cast<int>(value);
+    return OMX_OK;
+  }
   if (name && strcmp(name, "flash_kv_parts") == 0) {
     if (value < 0 || value > 64) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: flash_kv_parts takes 0..64");
     ctx->flash_kv_parts = static_cast<int>(value);

@@ -237,11 +237,12 @@ __device__ __forceinline__ bool at_store(float* row, const floatx4_a (&out)[AtDi
 struct AtPlace {
   int block, plane;
 };
-__device__ __forceinline__ AtPlace at_place() {
-  const unsigned planes = gridDim.y, share = min(8u, planes & (0u - planes));
-  const unsigned index = blockIdx.y * gridDim.x + blockIdx.x, n = index / share, run = n / gridDim.x;
-  return {static_cast<int>(n - run * gridDim.x), static_cast<int>(index % share + share * run)};
+__device__ __forceinline__ AtPlace at_place(unsigned index, unsigned blocks, unsigned planes) {
+  const unsigned share = min(8u, planes & (0u - planes));
+  const unsigned n = index / share, run = n / blocks;
+  return {static_cast<int>(n - run * blocks), static_cast<int>(index % share + share * run)};
 }
+__device__ __forceinline__ AtPlace at_place() { return at_place(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x, gridDim.y); }
 // Where part blockIdx.z of a row's result goes (Sdpa32Args::partial).
 __device__ __forceinline__ float* at_partial(const Sdpa32Args& a, int dim, int b, int kvh, int query, int head) {
   const long row = (static_cast<long>(b) * a.tq + query) * a.kv_heads * a.rep + static_cast<long>(kvh) * a.rep + head;
@@ -851,19 +852,19 @@ struct AtGrad {
 // second of their two rounds idle. At 152, without spills, they fit one: backward 58.8 -> 54.9 us
 // (360 rows, 32 planes 53.3 -> 49.7). At D = 128 a bound of two spills and costs 8-28 %: none there.
 template <int D, int KW>
-__global__ __launch_bounds__(AT_THREADS, D == 64 && KW == 4 ? 3 : 1) void sdpa32_dq_kernel(Sdpa32Args a) {
+constexpr int at_dq_lds() { return KW == 1 ? 2 * AT_ROWS * AtDim<D>::P : 4 * 16 * AtDim<D>::P; }
+template <int D, int KW>
+__device__ __forceinline__ void at_dq(const Sdpa32Args& a, AtPlace place, int blocks, float* lds) {
   using X = AtDim<D>;
   constexpr int QW = 4 / KW, BQ = 16 * QW, BLOCKS = KW == 1 ? 4 : 1, KEYS = 16 * BLOCKS;
-  __shared__ __align__(16) float lds[KW == 1 ? 2 * AT_ROWS * X::P : 4 * 16 * X::P];
   static_assert(16 * X::P >= X::S * 256, "the waves' sums fit");
   float* kt = lds;
   float* vt = lds + AT_ROWS * X::P;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int qw = wave % QW, kw = wave / QW;
-  const AtPlace place = at_place();
   const int b = place.plane / a.kv_heads, kvh = place.plane - b * a.kv_heads;
   const int rows = a.tq * a.rep;
-  const int r0 = (gridDim.x - 1 - place.block) * BQ;
+  const int r0 = (blocks - 1 - place.block) * BQ;
   const int r = r0 + qw * 16 + i;
   const AtRow at = at_unpack(min(r, rows - 1), a.rep);
   const long head = static_cast<long>(kvh) * a.rep + at.head;
@@ -989,23 +990,29 @@ __global__ __launch_bounds__(AT_THREADS, D == 64 && KW == 4 ? 3 : 1) void sdpa32
   }
   if (bad) dev_raise_fault(a.fault, a.tag);
 }
+template <int D, int KW>
+__global__ __launch_bounds__(AT_THREADS, D == 64 && KW == 4 ? 3 : 1) void sdpa32_dq_kernel(Sdpa32Args a) {
+  __shared__ __align__(16) float lds[at_dq_lds<D, KW>()];
+  at_dq<D, KW>(a, at_place(), static_cast<int>(gridDim.x), lds);
+}
 
 // dK and dV of 16 KG keys, over a share (blockIdx.z of gridDim.z) of the row tiles that see them.
 // Two workgroups per compute unit at D = 128, RW = 1 (LDS allows two; without the bound registers
 // allow one): 512 rows of 64 planes, backward 308 -> 278 us; 12 bytes of a lane go to scratch.
-template <int D, int RW>  // RW waves share a tile's rows, 4 / RW take 16 keys each
-__global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa32_dkv_kernel(Sdpa32Args a) {
+// OWN: each row's delta is formed here, from `out`, and not read from what the dQ pass left (RW = 4).
+template <int D, int RW>
+constexpr int at_dkv_lds() { return RW == 1 ? 2 * AT_ROWS * AtDim<D>::P + 2 * AT_ROWS : 4 * 2 * 16 * AtDim<D>::P; }
+template <int D, int RW, bool OWN>  // RW waves share a tile's rows, 4 / RW take 16 keys each
+__device__ __forceinline__ void at_dkv(const Sdpa32Args& a, AtPlace place, int part, int parts, int planes, float* lds) {
   using X = AtDim<D>;
   // RW = 4: nothing but the waves' sums goes through LDS; row tiles are blocks of 16 rows.
   constexpr int KG = 4 / RW, BK = 16 * KG, NB = AT_ROWS / 16, ROWS = RW == 1 ? AT_ROWS : 16;
-  __shared__ __align__(16) float lds[RW == 1 ? 2 * AT_ROWS * X::P + 2 * AT_ROWS : 4 * 2 * 16 * X::P];
   float* qt = lds;
   float* gt = lds + AT_ROWS * X::P;
   float* lse_t = gt + AT_ROWS * X::P;
   float* delta_t = lse_t + AT_ROWS;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), i = lane & 15, g = lane >> 4;
   const int kg = wave % KG, rw = wave / KG;
-  const AtPlace place = at_place();
   const int b = place.plane / a.kv_heads, kvh = place.plane - b * a.kv_heads;
   const int rows = a.tq * a.rep;
   const int j0 = place.block * BK, key = j0 + kg * 16 + i;
@@ -1017,8 +1024,8 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
   const int key_last = min(j0 + BK, a.tk) - 1;
   const int q_last = a.window > 0 ? min(a.tk - 1, key_last + a.window - 1) : a.tk - 1;
   const int u_first = j0 * a.rep / ROWS, u_end = ((q_last + 1) * a.rep + ROWS - 1) / ROWS;
-  const int share = (u_end - u_first + gridDim.z - 1) / gridDim.z;
-  const int u0 = u_first + blockIdx.z * share, u1 = min(u_end, u0 + share);
+  const int share = (u_end - u_first + parts - 1) / parts;
+  const int u0 = u_first + part * share, u1 = min(u_end, u0 + share);
   const long stat_b = (static_cast<long>(b) * a.kv_heads + kvh) * a.rep;
   const float* qb = a.q + b * a.q_b + static_cast<long>(kvh) * a.rep * a.q_h;
   const float* gb = a.gy + b * a.o_b + static_cast<long>(kvh) * a.rep * a.o_h;
@@ -1085,7 +1092,8 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
     // A block comes straight into the first two products' operands, a block ahead (a whole one where there are registers for
     // two); the other form goes through LDS of the wave's own.
     constexpr int SETS = D <= 64 ? 2 : 1;
-    AtDotBlock<D, float> qn[SETS], gn[SETS];
+    AtDotBlock<D, float> qn[SETS], gn[SETS], on[OWN ? SETS : 1];
+    const float* ob = OWN ? a.out + b * a.o_b + static_cast<long>(kvh) * a.rep * a.o_h : nullptr;
     float lse_n[SETS][4], delta_n[SETS][4];
     float* const own_q = lds + rw * (2 * 16 * X::P);
     float* const own_g = own_q + 16 * X::P;
@@ -1118,10 +1126,11 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
       }
       qn[set].fetch(at_bytes(qb + query0 * a.q_t), q_off);
       gn[set].fetch(at_bytes(gb + query0 * a.o_t), g_off);
+      if constexpr (OWN) on[set].fetch(at_bytes(ob + query0 * a.o_t), g_off);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         lse_n[set][j] = at_load<float>(at_bytes(a.lse + stat_b * a.tq + query0), stat[j]);
-        delta_n[set][j] = at_load<float>(at_bytes(a.delta + stat_b * a.tq + query0), stat[j]);
+        if constexpr (!OWN) delta_n[set][j] = at_load<float>(at_bytes(a.delta + stat_b * a.tq + query0), stat[j]);
       }
     };
     auto step = [&](int set, int u_now) {
@@ -1134,10 +1143,17 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
       if constexpr (SETS == 2) fetch(set ^ 1, min(u_now + RW, u1 - 1));
       const floatx4_a s = qn[set].dot(k), dp = gn[set].dot(v4);
       float lv[4], dl[4];
+      float row = 0.0f;  // delta of row i, as the dQ pass sums it
+      if constexpr (OWN) {
+#pragma unroll
+        for (int n = 0; n < X::S; ++n)
+          row += gn[set].raw[n][0] * on[set].raw[n][0] + gn[set].raw[n][1] * on[set].raw[n][1] + gn[set].raw[n][2] * on[set].raw[n][2] + gn[set].raw[n][3] * on[set].raw[n][3];
+        row = at_row_sum(row);
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         lv[j] = lse_n[set][j] * AT_LOG2E;
-        dl[j] = delta_n[set][j];
+        dl[j] = OWN ? __shfl(row, 4 * g + j) : delta_n[set][j];
       }
       if constexpr (SETS == 1) fetch(set, min(u_now + RW, u1 - 1));
       // Without masks where the block's first and last queries see every key (uniform).
@@ -1170,11 +1186,11 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
     }
     bad |= check != 0.0f;
   }
-  const bool split = gridDim.z > 1;
+  const bool split = parts > 1;
   const long plane = static_cast<long>(a.tk) * D;  // parts: [z][b, kv head][tk][D], dK's then dV's
-  const long part_at = ((static_cast<long>(blockIdx.z) * gridDim.y + place.plane) * a.tk + min(key, a.tk - 1)) * D;
+  const long part_at = ((static_cast<long>(part) * planes + place.plane) * a.tk + min(key, a.tk - 1)) * D;
   float* ok = split ? a.parts + part_at : a.gk + k_at;
-  float* ov = split ? a.parts + static_cast<long>(gridDim.z) * gridDim.y * plane + part_at : a.gv + k_at;
+  float* ov = split ? a.parts + static_cast<long>(parts) * planes * plane + part_at : a.gv + k_at;
   if constexpr (RW == 1) {
     if (key < a.tk) {
       bad |= at_store<D, 4>(ok, dk, 1.0f, g, 0);
@@ -1204,6 +1220,24 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
     }
   }
   if (bad) dev_raise_fault(a.fault, a.tag);
+}
+template <int D, int RW>
+__global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa32_dkv_kernel(Sdpa32Args a) {
+  __shared__ __align__(16) float lds[at_dkv_lds<D, RW>()];
+  at_dkv<D, RW, false>(a, at_place(), static_cast<int>(blockIdx.z), static_cast<int>(gridDim.z), static_cast<int>(gridDim.y), lds);
+}
+
+// Both passes in one launch (at_bwd_together says when): the key side's workgroups, a part after the other, then the dQ pass's.
+template <int D>
+__global__ __launch_bounds__(AT_THREADS, 2) void sdpa32_bwd_kernel(Sdpa32Args a, unsigned planes, unsigned row_blocks, unsigned key_blocks, unsigned parts) {
+  __shared__ __align__(16) float lds[at_dkv_lds<D, 4>() > at_dq_lds<D, 4>() ? at_dkv_lds<D, 4>() : at_dq_lds<D, 4>()];
+  const unsigned each = key_blocks * planes, keys = each * parts;
+  if (blockIdx.x < keys) {
+    const unsigned part = blockIdx.x / each;
+    at_dkv<D, 4, true>(a, at_place(blockIdx.x - part * each, key_blocks, planes), static_cast<int>(part), static_cast<int>(parts), static_cast<int>(planes), lds);
+  } else {
+    at_dq<D, 4>(a, at_place(blockIdx.x - keys, row_blocks, planes), static_cast<int>(row_blocks), lds);
+  }
 }
 
 // Adds up the parts of a split key / value pass, lowest rows first. blockIdx.y: 0 dK, 1 dV.
@@ -1239,6 +1273,33 @@ bool at_narrow(omx_ctx* ctx, const Sdpa32Args& a, long planes, long rows, long s
 }
 // What one row's, or key's, other side comes to.
 long at_span(const Sdpa32Args& a) { return a.window > 0 ? std::min<long>(a.tk, a.window + 15l) : a.tk; }
+
+// Whether the two passes of the backward share a launch (16-row and 16-key workgroups of head_dim up to 64, the output at hand). The key side
+// then forms delta itself, from the output's rows beside the gradient's, and nothing waits for the dQ pass: its workgroups
+// fill in where the longer ones of the key side, which go out first, leave room. Every bit is the same. us of a backward, two launches / one (head
+// dim 64): 2 x 8 over 2 x 777 in a window of 256: 54 / 44; the same without: 74 / 66; 1 x 4 x 128: 13.6 / 8.2; 8 x 4 x 256: 30 / 27;
+// 4 over 1 x 1500: 79 / 65; 2 x 12 x 1024: 152 / 150; 2 x 2048: 78 / 83; 16 x 4096: 1125 / 1238; 2 x 8 x 500 x 16: 20 / 15.
+// Gradients over what the other pass still reads (keys and values, or the output) take two launches, as they always could.
+bool at_bwd_together(omx_ctx* ctx, const Sdpa32Args& a, int planes, int dim) {
+  if (!a.out || (ctx->attention_together >= 0 ? ctx->attention_together == 0 : at_span(a) > 1536)) return false;
+  struct Range {
+    const char *first, *end;
+  };
+  const long batches = planes / a.kv_heads, heads = static_cast<long>(a.kv_heads) * a.rep;
+  auto range = [&](const void* p, long b, long h, long t, long n, long rows) {
+    const char* first = static_cast<const char*>(p);
+    return Range{first, first + 4 * ((batches - 1) * b + (n - 1) * h + (rows - 1) * t + dim)};
+  };
+  const Range read[] = {range(a.q, a.q_b, a.q_h, a.q_t, heads, a.tq), range(a.k, a.k_b, a.k_h, a.k_t, a.kv_heads, a.tk),
+                        range(a.v, a.k_b, a.k_h, a.k_t, a.kv_heads, a.tk), range(a.out, a.o_b, a.o_h, a.o_t, heads, a.tq),
+                        range(a.gy, a.o_b, a.o_h, a.o_t, heads, a.tq)};
+  const Range written[] = {range(a.gq, a.q_b, a.q_h, a.q_t, heads, a.tq), range(a.gk, a.k_b, a.k_h, a.k_t, a.kv_heads, a.tk),
+                           range(a.gv, a.k_b, a.k_h, a.k_t, a.kv_heads, a.tk)};
+  for (const Range& r : read)
+    for (const Range& w : written)
+      if (r.first < w.end && w.first < r.end) return false;
+  return true;
+}
 
 // sdpa_prompt_kernel: bf16 caches of wider heads, unless a ring's rows lie past 32 bits of lane offset from its first (4 GiB and
 // more of one batch entry's keys) and the keys that are read run past its end.
@@ -1286,14 +1347,8 @@ int32_t forward(omx_ctx* ctx, const Sdpa32Args& a, int planes, bool bf16_cache) 
 template <int D>
 int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
   const long rows = static_cast<long>(a.tq) * a.rep;
-  {
-    const bool narrow = at_narrow(ctx, a, planes, rows, at_span(a));
-    const long bq = narrow ? 16 : 64;
-    dim3 grid(static_cast<unsigned>((rows + bq - 1) / bq), planes);
-    if (narrow) omx_launch(ctx, (sdpa32_dq_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
-    else omx_launch(ctx, (sdpa32_dq_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);
-    OMX_LAUNCH_CHECK(ctx, "sdpa32_dq_kernel");
-  }
+  const bool row_narrow = at_narrow(ctx, a, planes, rows, at_span(a));
+  const long bq = row_narrow ? 16 : 64, row_blocks = (rows + bq - 1) / bq;
   const bool narrow = at_narrow(ctx, a, planes, a.tk, at_span(a) * a.rep);
   const long bk = narrow ? 16 : 64, blocks = (a.tk + bk - 1) / bk;
   // Into how many parts the rows are split: two workgroups per compute unit or more, as long as a share keeps two tiles of 64. Under the
@@ -1317,10 +1372,22 @@ int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
   // (as many as there is room for, down to one workgroup's walk over all rows)
   for (; parts > 1; --parts)
     if ((a.parts = static_cast<float*>(omx_workspace_if_room(ctx, static_cast<uint64_t>(parts) * total * 8, 1)))) break;
-  dim3 grid(static_cast<unsigned>(blocks), planes, static_cast<unsigned>(parts));
-  if (narrow) omx_launch(ctx, (sdpa32_dkv_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
-  else omx_launch(ctx, (sdpa32_dkv_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);
-  OMX_LAUNCH_CHECK(ctx, "sdpa32_dkv_kernel");
+  // In one launch where the other side is short enough for the ends of two to weigh more than the third workgroup per compute unit that the
+  // dQ pass has alone (at_bwd_together).
+  if (D <= 64 && narrow && row_narrow && at_bwd_together(ctx, a, planes, D)) {
+    if constexpr (D <= 64)
+      omx_launch(ctx, sdpa32_bwd_kernel<D>, dim3(static_cast<unsigned>((row_blocks + blocks * parts) * planes)), dim3(AT_THREADS), 0, a, static_cast<unsigned>(planes),
+                 static_cast<unsigned>(row_blocks), static_cast<unsigned>(blocks), static_cast<unsigned>(parts));
+    OMX_LAUNCH_CHECK(ctx, "sdpa32_bwd_kernel");
+  } else {
+    const dim3 row_grid(static_cast<unsigned>(row_blocks), planes), grid(static_cast<unsigned>(blocks), planes, static_cast<unsigned>(parts));
+    if (row_narrow) omx_launch(ctx, (sdpa32_dq_kernel<D, 4>), row_grid, dim3(AT_THREADS), 0, a);
+    else omx_launch(ctx, (sdpa32_dq_kernel<D, 1>), row_grid, dim3(AT_THREADS), 0, a);
+    OMX_LAUNCH_CHECK(ctx, "sdpa32_dq_kernel");
+    if (narrow) omx_launch(ctx, (sdpa32_dkv_kernel<D, 4>), grid, dim3(AT_THREADS), 0, a);
+    else omx_launch(ctx, (sdpa32_dkv_kernel<D, 1>), grid, dim3(AT_THREADS), 0, a);
+    OMX_LAUNCH_CHECK(ctx, "sdpa32_dkv_kernel");
+  }
   if (parts > 1) {
     omx_launch(ctx, sdpa32_parts_kernel, dim3(static_cast<unsigned>((total / 4 + AT_THREADS - 1) / AT_THREADS), 2), dim3(AT_THREADS), 0, a, static_cast<int>(parts), D, total);
     OMX_LAUNCH_CHECK(ctx, "sdpa32_parts_kernel");

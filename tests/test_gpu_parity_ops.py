@@ -526,6 +526,33 @@ def test_causal_sdpa_f32_tiled_kernels_agree_with_the_row_kernels(be, shape, hkv
             close(a, c, F32_TOL, "tiled against the oracle: " + name)
 
 
+@pytest.mark.parametrize("shape,hkv,window", [((1, 1, 1, 64), 1, None), ((2, 8, 97, 64), 2, 33), ((1, 3, 130, 16), 1, None), ((3, 5, 77, 32), 5, 20),
+                                              ((1, 4, 1537, 64), 2, None), ((1, 3, 33, 64), 1, None)])
+def test_f32_attention_backward_in_one_launch_has_the_bits_of_two(be, shape, hkv, window):
+    """Both passes of the f32 backward in one launch, the key side's row terms formed there: every bit of two launches, groups whose
+    rows do and do not lie in order and row blocks past the end among them. Gradients in place of keys and values, which the other pass reads."""
+    from ojas_amd.backend import F32, _native
+
+    b, h, t, d = shape
+    rng = np.random.default_rng(t)
+    x = [be.upload(rng.normal(size=(b, n, t, d)).astype(np.float32)) for n in (h, hkv, hkv, h)]
+    y, lse = be.causal_sdpa_forward(*x[:3], window, F32)
+    got = {}
+    try:
+        for together in (0, 1):
+            be.set_option("attention_together", together)
+            got[together] = [be.download(g) for g in be.causal_sdpa_backward(*x[:3], y, lse, x[3], window, F32)]
+        for two, one in zip(got[0], got[1]):
+            np.testing.assert_array_equal(one, two)
+        gq = be.empty(shape)
+        _native.omx_causal_sdpa_backward(be._context, x[0], x[1], x[2], y, lse, x[3], F32, F32, F32, gq, x[1], x[2], F32, b, h, hkv, t, d,
+                                         window or 0)
+        for g, e in zip((gq, x[1], x[2]), got[0]):
+            np.testing.assert_array_equal(be.download(g), e)
+    finally:
+        be.set_option("attention_together", -1)
+
+
 @pytest.mark.parametrize("b,h,hkv,t,d,window,tiled", [(2, 4, 2, 70, 64, 0, 0), (1, 3, 3, 130, 16, 40, 0), (2, 2, 1, 65, 128, 0, 0),
                                                     (16500, 4, 4, 3, 16, 0, 1), (8200, 8, 8, 2, 32, 1, 1)])
 def test_time_major_f32_attention_takes_the_row_kernels_where_it_must(be, b, h, hkv, t, d, window, tiled):
