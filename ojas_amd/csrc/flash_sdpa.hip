@@ -785,9 +785,10 @@ struct DkvHalf {
 // take more than 256 registers, so one wave has its SIMD to itself, and everything it waits for has to be on its way: tiles go straight
 // into LDS a tile ahead, operands come from LDS a phase ahead (DkvHalf), rows go out whole lines at a time.
 // What bounds it: products and vector work, which do not overlap, about 0.6 of the time; then the first tile and the last rows (5 us a
-// workgroup at 128). us, through registers (two walks at 128, scores formed twice) / now: 4 x 16 x 2048 x 128: 220 / 159; 8 x 16 x 1024 x
-// 128: 143 / 106; 16 x 12 x 1024 x 64: 85 / 70; 8 x 12 x 1024 x 64: 47 / 41. Waiting for a tile, storing it and asking for the next were
-// 1500 of 5900 clocks a tile, the waits for operands 1000.
+// workgroup at 128). us, through registers (two walks at 128, scores formed twice) / now: 4 x 16 x 2048 x 128: 221 / 168; 8 x 16 x 1024 x
+// 128: 141 / 110; 16 x 12 x 1024 x 64: 83 / 74; 8 x 12 x 1024 x 64: 46 / 42. Waiting for a tile, storing it and asking for the next were
+// 1500 of 5900 clocks a tile, the waits for operands 1000. Scores and dP from accumulators that start at the rows' values would save a
+// subtraction each (159 and 70 us), in other roundings.
 // GROUPS > 1: groups of the waves take the query tiles of 128 / GROUPS keys in turn, as in the forward.
 // SPLIT: the tiles of s.kv_parts workgroups are consecutive shares of the sequence over the heads, this one's is `part`, and its sums go
 // out as rows of gk and gv, each [part][b, KV head][time][D].
@@ -939,12 +940,11 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     for (int j = 0; j < GROUPS; ++j) turn();
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();  // the last loads into LDS are done
+  __syncthreads();  // every wave is done with the tiles, the last loads into LDS with them
   bool bad = false;
   if constexpr (GROUPS > 1) {
     constexpr int PART = 2 * MT * 16 * 64;  // floats of a wave
     float* const meet = reinterpret_cast<float*>(lds);
-    __syncthreads();  // every wave is done with the tiles
     if (group > 0) {
       float* mine = meet + ((group - 1) * ROW_WAVES + wave) * PART + lane;
 #pragma unroll
@@ -956,8 +956,9 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
         }
     }
     __syncthreads();
+    if (group > 0) return bad;
 #pragma unroll
-    for (int g = 0; g < (group > 0 ? 0 : GROUPS - 1); ++g) {
+    for (int g = 0; g < GROUPS - 1; ++g) {
       const float* part = meet + (g * ROW_WAVES + wave) * PART + lane;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
@@ -967,13 +968,16 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
           dv[mt][vv] += part[(MT * 16 + mt * 16 + vv) * 64];
         }
     }
-    __syncthreads();  // (read before the rows go out through the same memory)
-    if (group > 0) return bad;
   }
   const long out_off = SPLIT ? ((static_cast<long>(part) * s.batch + b) * s.kv_heads + gidx) * T * D : kv_off, out_rs = SPLIT ? D : s.kv.rs;
-  char* const stage = lds + wave * (32 * D * static_cast<int>(sizeof(TO)));
-  bad |= store_acc_rows<D, TO>(gk + out_off, out_rs, wave_k0, T, lane, dk, s.scale, stage);
-  bad |= store_acc_rows<D, TO>(gv + out_off, out_rs, wave_k0, T, lane, dv, 1.0f, stage);
+  if constexpr (GROUPS > 1) {  // (whole lines, by way of LDS, would wait for it once more and cost 0.5 to 1 us here)
+    bad |= store_transposed_acc<D, TO>(gk + out_off, out_rs, key_row, T, lg, dk, s.scale);
+    bad |= store_transposed_acc<D, TO>(gv + out_off, out_rs, key_row, T, lg, dv, 1.0f);
+  } else {
+    char* const stage = lds + wave * (32 * D * static_cast<int>(sizeof(TO)));
+    bad |= store_acc_rows<D, TO>(gk + out_off, out_rs, wave_k0, T, lane, dk, s.scale, stage);
+    bad |= store_acc_rows<D, TO>(gv + out_off, out_rs, wave_k0, T, lane, dv, 1.0f, stage);
+  }
   return bad;
 }
 
@@ -1416,14 +1420,14 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
   for_groups<D>(groups, with_groups);
 }
 
-// How the key side's pass is cut: groups of waves that take a key block's query tiles in turn, and parts, consecutive shares of those
-// tiles on workgroups of their own, whose f32 sums go through scratch to a second launch that adds them in order. The pass has a
+// How the key side's pass is cut: groups of waves that take a key block's query tiles in turn (flash_groups), and parts, consecutive shares of
+// those tiles on workgroups of their own, whose f32 sums go through scratch to a second launch that adds them in order. The pass has a
 // workgroup per key block and KV head, so few KV heads leave units idle however many query heads there are, and a workgroup walks the
-// tiles of all of them, 1.3 to 1.7 us apiece. The estimate is the root of the squares of the longest walk and of the chip's work, per
-// key block of 128, 64 or 32 keys, fitted to 24 shapes x 3 group counts x 8 part counts (rms 6 to 12 %); the second launch takes 4.5 us
-// or 2 us and 0.14 us a megabyte. Parts are taken where they gain a twentieth. Over those shapes the choice takes 2.5 % more than the
-// best of all counts on average, 12 % at most. us of the pass, one group and part / by the rule: 10 x 13 heads over one x 670: 201 /
-// 43; 2 x 8 over 2 x 1024 x 128: 114 / 35; 8 over 2 x 291 x 128: 51 / 27; 12 x 2048: 42 / 31; 8 x 1024: 24 / 15; many planes (8 x 12
+// tiles of all of them, 1.3 to 1.9 us apiece. Parts are taken where an estimate says that they gain a tenth: the root of the squares of the
+// longest walk and of the chip's work, per key block of 128, 64 or 32 keys, fitted to 32 shapes x 3 group counts x 8 part counts (rms 9
+// to 12 %); the second launch takes 4.5 us or 2 us and 0.14 us a megabyte. Over those shapes the choice takes 1.5 % more than the
+// best of all counts on average, 13 % at most. us of the pass, one group and part / by the rule: 10 x 13 heads over one x 670: 207 /
+// 45; 2 x 8 over 2 x 1024 x 128: 125 / 38; 8 over 2 x 291 x 128: 54 / 29; 12 x 2048: 43 / 31; 8 x 1024: 25 / 15; many planes (8 x 12
 // x 1024: 44) stay whole.
 struct FlashKeyPlan {
   int groups, parts, whole_groups;  // whole_groups: without parts
@@ -1434,15 +1438,16 @@ FlashKeyPlan flash_key_plan(omx_ctx* ctx, const FlashShape& s, int dim) {
     const int groups = ctx->flash_schedule < 3 ? 1 : std::min(dim == 64 ? 4 : 2, ctx->flash_schedule == 3 ? 2 : 4);
     return {groups, std::max(1, ctx->flash_kv_parts), groups};
   }
-  if (planes * ((s.time + 127) / 128) >= 2 * units) return {1, std::max(1, ctx->flash_kv_parts), 1};
+  const int whole_groups = flash_groups(ctx, static_cast<unsigned>(planes), s.time, static_cast<int>(std::min<long>(static_cast<long>(flash_tiles(s)) * s.rep, 1 << 20)),
+                                        s.window > 0, dim);
+  if (ctx->flash_kv_parts || planes * ((s.time + 127) / 128) >= 2 * units) return {whole_groups, std::max(1, ctx->flash_kv_parts), whole_groups};
   struct Fit {
     double first, step, work, each;  // us: of a workgroup, of a tile on its way; of a unit's tiles, of a unit's workgroups
   };
-  const Fit fits[2][3] = {{{10.1, 1.27, 0.59, 4.03}, {10.4, 1.36, 0.86, 4.05}, {9.7, 1.72, 1.61, 8.17}},
-                          {{13.2, 1.53, 1.45, 9.4}, {15.2, 1.54, 1.50, 10.9}, {}}};
+  const Fit fits[2][3] = {{{9.5, 1.33, 0.60, 4.2}, {9.4, 1.42, 0.83, 4.0}, {8.7, 1.81, 1.55, 7.55}}, {{13.2, 1.82, 1.85, 9.6}, {13.6, 1.90, 1.92, 10.0}, {}}};
   const double megabytes = 8e-6 * static_cast<double>(planes) * s.time * dim;
   double whole = 1e30, least = 1e30;
-  FlashKeyPlan plan = {1, 1, 1};
+  FlashKeyPlan plan = {whole_groups, 1, whole_groups};
   for (int shift = 0; shift < (dim == 64 ? 3 : 2); ++shift) {
     const int g = 1 << shift, rows = 128 / g, blocks = (s.time + rows - 1) / rows;
     const Fit& f = fits[dim == 128][shift];
@@ -1459,10 +1464,7 @@ FlashKeyPlan flash_key_plan(omx_ctx* ctx, const FlashShape& s, int dim) {
       const double walk = f.first + f.step * static_cast<double>((most + p * g - 1) / (p * g));
       const double work = f.work * (static_cast<double>(all * planes) / static_cast<double>(g * units) + (p * g > 1 ? 0.5 * groups_of_units : 0.0)) + f.each * groups_of_units;
       const double us = std::sqrt(walk * walk + work * work) + (p > 1 ? std::max(4.5, 2.0 + 0.14 * megabytes * p) : 0.0);
-      if (p == 1 && us < whole) {
-        whole = us;
-        plan.whole_groups = g;
-      }
+      if (p == 1) whole = std::min(whole, us);
       if (p > 1 && us < least) {
         least = us;
         plan.groups = g;
@@ -1470,8 +1472,7 @@ FlashKeyPlan flash_key_plan(omx_ctx* ctx, const FlashShape& s, int dim) {
       }
     }
   }
-  if (least >= 0.95 * whole) plan = {plan.whole_groups, 1, plan.whole_groups};
-  if (ctx->flash_kv_parts) plan = {plan.whole_groups, ctx->flash_kv_parts, plan.whole_groups};
+  if (least >= 0.9 * whole) plan = {whole_groups, 1, whole_groups};
   return plan;
 }
 
