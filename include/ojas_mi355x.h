@@ -585,6 +585,14 @@ int32_t omx_swiglu_forward(omx_ctx* ctx, const void* gate_up, void* out, int32_t
                            uint64_t hidden);
 int32_t omx_swiglu_backward(omx_ctx* ctx, const void* gate_up, const void* gy, void* g_gate_up,
                             int32_t dtype, uint64_t rows, uint64_t hidden);
+/* linear_forward (backend.rs:1628-1645) of a fused gate | up projection, w [2 hidden, in] with the gate rows first, and swiglu_forward of
+ * what it leaves, every bit as those two calls have it: gate_up [rows, 2 hidden] of `gate_up_dtype`, out [rows, hidden] bf16. The second
+ * form over int8 codes (omx_linear_i8_group_forward, gate_up f32). */
+int32_t omx_linear_swiglu_forward(omx_ctx* ctx, const void* x, const void* w, int32_t operand_dtype, void* gate_up, int32_t gate_up_dtype,
+                                  void* out, uint64_t rows, uint64_t in_features, uint64_t hidden);
+int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32,
+                                           uint64_t group, int32_t layout, void* gate_up, void* out, uint64_t rows, uint64_t kin,
+                                           uint64_t hidden);
 /* Synthetic weights made on the device (no counterpart in the reference, whose init runs on the
  * host, ojas-model/src/init.rs:67-114): element i is N(0, std) from a counter-based generator of
  * (seed, i). omx_init_normal_i8_group draws row-major [n_out, k_in] values and stores them

@@ -589,7 +589,11 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   // GELU in f32: in the store pass of the kernels that have one (gemm_dma32_kernel, A k-contiguous), else a pass of its own after it.
   const OmxGemmEpilogue* act32 = epi && (epi->mode == OMX_EPI_GELU_FWD || epi->mode == OMX_EPI_GELU_BWD) && operand_dtype == OMX_F32 &&
                                          c_dtype == OMX_F32 && !accumulate && batches == 1 && ldc == n ? epi : nullptr;
-  if (sum32 || act32) epi = nullptr;
+  // Gates and ups of one product (OMX_EPI_SWIGLU): on the 256 x 256 one-wave kernel in its store pass, otherwise a pass after it.
+  const OmxGemmEpilogue* swiglu = epi && epi->mode == OMX_EPI_SWIGLU ? epi : nullptr;
+  if (swiglu && (operand_dtype != OMX_BF16 || c_dtype != OMX_F32 || accumulate || batches != 1 || low_rank || ldc != n || n % 2 != 0))
+    return omx_fail(ctx, OMX_UNSUPPORTED, "%s: gates and ups go with one plain bf16 product into f32", op);
+  if (sum32 || act32 || swiglu) epi = nullptr;
   if (epi && epi->mode != OMX_EPI_NONE && c_dtype != OMX_BF16)
     return omx_fail(ctx, OMX_DTYPE, "%s: a fused activation needs a bf16 output", op);
   if (!a || !b || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
@@ -801,17 +805,22 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       ctx->gemm_in_row_split = true;
       ctx->gemm_forced_tiling = dma_variant;
       int32_t rc = omx_gemm_impl(ctx, fault_op, a, a_rs, a_cs, b, b_rs, b_cs, operand_dtype, c, c_dtype, ldc, m0, k, n,
-                                 accumulate, epi, nullptr, a_k, low_rank);
+                                 accumulate, swiglu ? swiglu : epi, nullptr, a_k, low_rank);
       ctx->gemm_forced_tiling = -1;
       OmxLowRank rest_rank{};
       if (low_rank) {
         rest_rank = *low_rank;
         rest_rank.h = static_cast<const unsigned short*>(rest_rank.h) + m0 * rest_rank.h_pitch;
       }
+      OmxGemmEpilogue rest_pairs{};
+      if (swiglu) {
+        rest_pairs = *swiglu;
+        rest_pairs.aux_out = static_cast<unsigned short*>(swiglu->aux_out) + m0 * (n / 2);
+      }
       if (rc == OMX_OK)
         rc = omx_gemm_impl(ctx, fault_op, static_cast<const char*>(a) + m0 * a_rs * esz, a_rs, a_cs, b, b_rs, b_cs,
                            operand_dtype, static_cast<char*>(c) + m0 * ldc * csz, c_dtype, ldc, m - m0, k, n,
-                           accumulate, epi, nullptr, a_k, low_rank ? &rest_rank : nullptr);
+                           accumulate, swiglu ? &rest_pairs : epi, nullptr, a_k, low_rank ? &rest_rank : nullptr);
       ctx->gemm_in_row_split = false;
       return rc;
     }
@@ -919,9 +928,17 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     g.aux_out = static_cast<unsigned short*>(act32->aux_out);
     if (!aligned16(act32->mode == OMX_EPI_GELU_FWD ? act32->aux_out : act32->aux_in)) g.c_vec = 0;
   }
+  // (a wave's 64 units are whole, and the lane offsets of a tile's rows, as far apart as gates and ups, stay within 31 bits of bytes)
+  const bool pairs_fused = swiglu && dma_variant == 9 && !a_km && !b_km && g.splits == 1 && n % 128 == 0 && g.c_vec && aligned16(swiglu->aux_out) &&
+                           (static_cast<long>(n) / 2 + 256) * ldb < (1l << 30);
+  if (pairs_fused) {
+    g.epi = OMX_EPI_SWIGLU;
+    g.aux_out = static_cast<unsigned short*>(swiglu->aux_out);
+  }
   g.fault = ctx->fault;
   g.tag = omx_tag(ctx, fault_op);
-  g.act_tag = act_fused ? omx_tag(ctx, act32->mode == OMX_EPI_GELU_FWD ? F_GELU_FORWARD : F_GELU_BACKWARD) : g.tag;
+  if (pairs_fused) g.act_tag = omx_tag(ctx, F_MUL_FORWARD);
+  else g.act_tag = act_fused ? omx_tag(ctx, act32->mode == OMX_EPI_GELU_FWD ? F_GELU_FORWARD : F_GELU_BACKWARD) : g.tag;
   omx_ctx::TimedLaunch timed{};
   if (ctx->profile_gemm) {
     auto take = [&](hipEvent_t* e) -> hipError_t {
@@ -966,6 +983,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     ctx->timing_start = ctx->timing_stop = nullptr;
     if (rc == OMX_OK) ctx->timed.push_back(timed);
   }
+  if (rc == OMX_OK && swiglu && !pairs_fused) rc = omx_swiglu_forward(ctx, c, swiglu->aux_out, OMX_F32, m, n / 2);
   if (rc == OMX_OK && act32 && !act_fused)
     rc = act32->mode == OMX_EPI_GELU_FWD ? omx_gelu_forward(ctx, c, act32->aux_out, OMX_F32, m * n, act32->tanh_form)
                                          : omx_gelu_backward(ctx, act32->aux_in, c, c, OMX_F32, m * n, act32->tanh_form);

@@ -513,7 +513,7 @@ bool widen_pays(const omx_ctx* ctx, uint64_t m, uint64_t k, uint64_t n) {
   return over_copy < 0.93 * over_codes;
 }
 int32_t widened_product(omx_ctx* ctx, uint32_t fault_op, const Q8Args& g, uint64_t rows, uint64_t kin, uint64_t nout,
-                        bool backward, bool* taken) {
+                        bool backward, bool* taken, const OmxGemmEpilogue* epi = nullptr) {
   *taken = false;
   const uint64_t k = backward ? nout : kin, n = backward ? kin : nout;
   constexpr uint64_t kMost = 1ull << 30;  // bytes of scratch
@@ -528,23 +528,17 @@ int32_t widened_product(omx_ctx* ctx, uint32_t fault_op, const Q8Args& g, uint64
                       static_cast<uint64_t>(g.lr_rank), static_cast<uint64_t>(g.lr_block_cols)};
   ctx->extra_in_use = true;
   const int32_t rc = omx_gemm_impl(ctx, fault_op, g.a, k, 1, w, backward ? kin : 1, backward ? 1 : kin, OMX_BF16, g.c,
-                                   g.c_f32 ? OMX_F32 : OMX_BF16, n, rows, k, n, 0, nullptr, nullptr, 0, g.lr_rank > 0 ? &lr : nullptr);
+                                   g.c_f32 ? OMX_F32 : OMX_BF16, n, rows, k, n, 0, epi, nullptr, 0, g.lr_rank > 0 ? &lr : nullptr);
   ctx->extra_in_use = false;
   // Partial sums that there is no room for: the codes' kernel has none.
   *taken = rc != OMX_CAPACITY_EXCEEDED;
   return *taken ? rc : OMX_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int32_t omx_linear_i8_group_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8,
-                                    const void* scales_f32, uint64_t group, int32_t layout, const void* add,
-                                    const omx_low_rank* low_rank, void* y, int32_t y_dtype, uint64_t rows,
-                                    uint64_t kin, uint64_t nout) {
-  OMX_REQUIRE_CTX(ctx);
-  const char* op = "linear_i8_group_forward";
+// `swiglu`: the products' columns are gates and ups, and their activation goes there (OMX_EPI_SWIGLU).
+int32_t i8_forward(omx_ctx* ctx, const char* op, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32, uint64_t group,
+                   int32_t layout, const void* add, const omx_low_rank* low_rank, void* y, int32_t y_dtype, uint64_t rows, uint64_t kin,
+                   uint64_t nout, void* swiglu) {
   int32_t rc = check_q8(ctx, op, x, codes_i8, scales_f32, y, add, rows, kin, nout, group, x_dtype, layout);
   if (rc != OMX_OK) return rc;
   if (!omx_valid_float_dtype(y_dtype)) return omx_fail(ctx, OMX_DTYPE, "%s: the output must be f32 or bf16", op);
@@ -569,10 +563,32 @@ int32_t omx_linear_i8_group_forward(omx_ctx* ctx, const void* x, int32_t x_dtype
   rc = set_low_rank(ctx, op, &g, low_rank, nout);
   if (rc != OMX_OK) return rc;
   bool taken = false;
-  rc = widened_product(ctx, F_LINEAR_FORWARD, g, rows, kin, nout, false, &taken);
+  const OmxGemmEpilogue pairs = {OMX_EPI_SWIGLU, 0, nullptr, swiglu};
+  rc = widened_product(ctx, F_LINEAR_FORWARD, g, rows, kin, nout, false, &taken, swiglu ? &pairs : nullptr);
   if (rc != OMX_OK || taken) return rc;
   g.tag = omx_tag(ctx, F_LINEAR_FORWARD);
-  return launch_q8<false>(ctx, g, 2.0 * rows * kin * nout);
+  rc = launch_q8<false>(ctx, g, 2.0 * rows * kin * nout);
+  return rc == OMX_OK && swiglu ? omx_swiglu_forward(ctx, y, swiglu, OMX_F32, rows, nout / 2) : rc;
+}
+
+}  // namespace
+
+extern "C" {
+
+int32_t omx_linear_i8_group_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8,
+                                    const void* scales_f32, uint64_t group, int32_t layout, const void* add,
+                                    const omx_low_rank* low_rank, void* y, int32_t y_dtype, uint64_t rows,
+                                    uint64_t kin, uint64_t nout) {
+  OMX_REQUIRE_CTX(ctx);
+  return i8_forward(ctx, "linear_i8_group_forward", x, x_dtype, codes_i8, scales_f32, group, layout, add, low_rank, y, y_dtype, rows, kin, nout, nullptr);
+}
+
+int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32, uint64_t group,
+                                           int32_t layout, void* gate_up, void* out, uint64_t rows, uint64_t kin, uint64_t hidden) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "linear_i8_group_swiglu_forward";
+  if (!out) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  return i8_forward(ctx, op, x, x_dtype, codes_i8, scales_f32, group, layout, nullptr, nullptr, gate_up, OMX_F32, rows, kin, 2 * hidden, out);
 }
 
 int32_t omx_linear_i8_group_backward_input(omx_ctx* ctx, const void* codes_i8, const void* scales_f32, uint64_t group,

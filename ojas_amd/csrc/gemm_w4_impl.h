@@ -49,6 +49,16 @@ struct W4Loads {
   static constexpr int N = ROWS / 32;  // ROWS / 8 loads of 1 KiB per step, four waves
   unsigned off[N];
   StepBase<KM, TAIL> base;
+  // Two row ranges, `half` apart, in one tile of 256: 64 rows of the first and the same of the second in turn. row0: of the first.
+  __device__ __forceinline__ void init_pairs(const unsigned short* __restrict__ p, long ld, int row0, int half, int k0, int k_rows, int wave, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = (wave + 4 * i) * 8 + (lane >> 3), kc = (lane & 7) ^ ((r >> 1) & 7);
+      const int unit = min(row0 + (r >> 7) * 64 + (r & 63), half - 1);
+      off[i] = static_cast<unsigned>(unit - row0 + (r >> 6 & 1) * half) * static_cast<unsigned>(ld * 2) + kc * 16;
+    }
+    base.init(p, ld, row0, k0, k_rows, W4_BK);
+  }
   __device__ __forceinline__ void init(const unsigned short* __restrict__ p, long ld, int row0, int rows, int k0,
                                        int k_rows, int wave, int lane) {
 #pragma unroll
@@ -122,10 +132,14 @@ struct W4Frags {
 };
 
 // LR: with a low-rank term.
-template <bool A_KM, bool B_KM, int TN, bool TAIL, bool LR = false>
+// PAIR: B's rows are gates and, N / 2 further, ups. A wave's 128 columns are 64 units' gates and ups, which meet in its store pass: C
+// as it would be, in f32, and silu(gate) up beside it in bf16 (OMX_EPI_SWIGLU), where a pass of its own read C again. us, product and pass / so,
+// inside a step: 8192 rows over 2048 -> 2 x 8192: 490 + 112 / 545; 16384 over 768 -> 2 x 2048: 130 + 59 / 154.
+template <bool A_KM, bool B_KM, int TN, bool TAIL, bool LR = false, bool PAIR = false>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   static_assert(!A_KM || B_KM, "a k-major A goes with a k-major B");
   static_assert(TN == 4 || TN == 3, "256 x 256 or 256 x 192 tiles");
+  static_assert(!PAIR || (!A_KM && !B_KM && TN == 4 && !TAIL && !LR), "one form of pairs");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr int TM = 4, NW = 4, W4_BN = TN * 64;
   // Tile order: as gemm_dma_kernel.
@@ -182,7 +196,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   W4Loads<A_KM, W4_BM, TAIL> la;
   W4Loads<B_KM, W4_BN, TAIL> lb;
   la.init(A, g.lda, m0, g.M, ks_begin * W4_BK, g.k_rows, wave, lane);
-  lb.init(B, g.ldb, n0, g.N, ks_begin * W4_BK, g.k_rows, wave, lane);
+  if constexpr (PAIR) lb.init_pairs(B, g.ldb, n0 / 2, g.N / 2, ks_begin * W4_BK, g.k_rows, wave, lane);
+  else lb.init(B, g.ldb, n0, g.N, ks_begin * W4_BK, g.k_rows, wave, lane);
   const unsigned lds_wave =
       __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem))) + wave * 1024;
   // Waits until at most YES (if `which`) or NO of this wave's loads, the most recently issued, are in flight.
@@ -441,11 +456,42 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   constexpr int HP = TN * 32 * 2 + 16;  // bytes per staged bf16 row
   char* hs = reinterpret_cast<char*>(cs);
   unsigned flags = 0;  // bit 15 or 31 set: a stored bf16 has an all-ones exponent
+  bool bad_act = false;
   static_for<0, TM>([&](auto tm_index) {
     constexpr int tm = decltype(tm_index)::value;
     const int grow0 = m0 + (wm * TM + tm) * 32;
     const bool interior = grow0 + 32 <= g.M && gcol0 + TN * 32 <= g.N;
-    if (packed && interior) {
+    if constexpr (PAIR) {
+      const int half = g.N / 2, unit0 = n0 / 2 + wn * 64;
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const floatx16& c = acc[tm][tn];
+          *reinterpret_cast<float4*>(cs + l32 * CPW + tn * 32 + 8 * q + 4 * lg) = make_float4(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]);
+        }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (unit0 < half) {  // (half is a multiple of 64)
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+          const int row = it * 4 + (lane >> 4), piece = (lane & 15) * 4;
+          const float4 gate = *reinterpret_cast<const float4*>(cs + row * CPW + piece), up = *reinterpret_cast<const float4*>(cs + row * CPW + 64 + piece);
+          if (grow0 + row < g.M) {
+            float* to = static_cast<float*>(g.c) + static_cast<long>(grow0 + row) * g.ldc + unit0 + piece;
+            *reinterpret_cast<float4*>(to) = gate;
+            *reinterpret_cast<float4*>(to + half) = up;
+            const float y0 = gate.x * dev_sigmoid(gate.x) * up.x, y1 = gate.y * dev_sigmoid(gate.y) * up.y, y2 = gate.z * dev_sigmoid(gate.z) * up.z,
+                        y3 = gate.w * dev_sigmoid(gate.w) * up.w;
+            *reinterpret_cast<uint2*>(g.aux_out + static_cast<long>(grow0 + row) * half + unit0 + piece) =
+                make_uint2(dev_pack_bf16_pair(y0, y1), dev_pack_bf16_pair(y2, y3));
+            bad |= !(dev_finite(gate.x) && dev_finite(gate.y) && dev_finite(gate.z) && dev_finite(gate.w) && dev_finite(up.x) && dev_finite(up.y) &&
+                     dev_finite(up.z) && dev_finite(up.w));
+            bad_act |= !(dev_finite(y0) && dev_finite(y1) && dev_finite(y2) && dev_finite(y3));
+          }
+        }
+      }
+    } else if (packed && interior) {
       // bf16: rounded in registers, staged 8 bytes at a time, stored 16 bytes per lane (a wave
       // instruction writes four rows of 64 TN bytes; with TN = 3 four lanes in 16 sit out).
 #pragma unroll
@@ -505,6 +551,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   });
   bad |= (flags & 0x80008000u) != 0;
   if (bad) dev_raise_fault(g.fault, g.tag);
+  if (PAIR && bad_act && !bad) dev_raise_fault(g.fault, g.act_tag);
 }
 
 template <bool A_KM, bool B_KM, int TN>
@@ -515,6 +562,9 @@ int32_t launch_w4(omx_ctx* ctx, const GemmArgs& g) {
   }
   if constexpr (!A_KM) {
     if (g.lr_rank > 0) kernel = &gemm_w4_kernel<A_KM, B_KM, TN, false, true>;  // (whole steps)
+  }
+  if constexpr (!A_KM && !B_KM && TN == 4) {
+    if (g.epi == OMX_EPI_SWIGLU) kernel = &gemm_w4_kernel<false, false, 4, false, false, true>;
   }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    W4_SMEM));

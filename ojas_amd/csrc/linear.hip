@@ -122,6 +122,22 @@ int32_t omx_linear_gelu_forward(omx_ctx* ctx, const void* x, const void* w, int3
                        out_features, rows, in_features, out_features, 0, &epi);
 }
 
+// A fused gate | up projection and its SwiGLU: gate_up [rows, 2 hidden] = x [w_gate; w_up]^T and out [rows, hidden] (bf16) = silu(gate) up.
+int32_t omx_linear_swiglu_forward(omx_ctx* ctx, const void* x, const void* w, int32_t operand_dtype, void* gate_up, int32_t gate_up_dtype, void* out,
+                                  uint64_t rows, uint64_t in_features, uint64_t hidden) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "linear_swiglu_forward";
+  if (!x || !w || !gate_up || !out) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (rows == 0 || in_features == 0 || hidden == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
+  if (operand_dtype == OMX_BF16 && gate_up_dtype == OMX_F32) {
+    OmxGemmEpilogue epi = {OMX_EPI_SWIGLU, 0, nullptr, out};
+    return omx_gemm_impl(ctx, F_LINEAR_FORWARD, x, in_features, 1, w, 1, in_features, operand_dtype, gate_up, OMX_F32, 2 * hidden, rows,
+                         in_features, 2 * hidden, 0, &epi);
+  }
+  const int32_t rc = omx_linear_forward(ctx, x, operand_dtype, w, operand_dtype, gate_up, gate_up_dtype, rows, in_features, 2 * hidden);
+  return rc == OMX_OK ? omx_swiglu_forward(ctx, gate_up, out, gate_up_dtype, rows, hidden) : rc;
+}
+
 // The input gradient of linear_backward followed by gelu_backward: gu = (gy W) * gelu'(u),
 // the derivative applied in the product's store pass. gy [rows, out], w [out, in], u / gu [rows, in].
 int32_t omx_linear_backward_input_gelu(omx_ctx* ctx, const void* w, const void* gy, int32_t operand_dtype,

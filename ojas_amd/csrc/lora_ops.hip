@@ -63,7 +63,6 @@ __global__ void rope_pitched_kernel(unsigned short* __restrict__ x, long pitch, 
   if (bad) dev_raise_fault(fault, tag);
 }
 
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
 // Eight consecutive values of a bf16 or an f32 tensor as floats (16-byte accesses).
 template <bool STREAM = false>
@@ -138,7 +137,7 @@ __global__ void swiglu_fwd_kernel(const GU* __restrict__ gate_up, unsigned short
   bool bad = false;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    y[e] = g[e] * sigmoid_f(g[e]) * u[e];
+    y[e] = g[e] * dev_sigmoid(g[e]) * u[e];
     bad |= !dev_finite(y[e]);
   }
   *reinterpret_cast<uint4*>(out + r * hidden + c) = pack8(y);
@@ -161,7 +160,7 @@ __global__ void swiglu_bwd_kernel(const GU* __restrict__ gate_up, const unsigned
   bool bad = false;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float s = sigmoid_f(g[e]);
+    const float s = dev_sigmoid(g[e]);
     gu[e] = d[e] * (g[e] * s);
     gg[e] = d[e] * u[e] * (s * (1.0f + g[e] * (1.0f - s)));
     bad |= !(dev_finite(gu[e]) && dev_finite(gg[e]));

@@ -236,8 +236,10 @@ inline unsigned long long omx_tag(omx_ctx* ctx, uint32_t op) {
 //   OMX_EPI_AXPBY: C = round_bf16(s1 aux_in) + round_bf16(s2 round_bf16(A.B)): the product stored as
 //     bf16, then the two-term sum a separate pass over it would form, in one store. f32 operands and output: C = s1 aux_in +
 //     s2 A.B, each term rounded as a pass of its own would.
+//   OMX_EPI_SWIGLU: C (f32, its first half of columns gates, the second ups) = A.B and aux_out [m, n / 2] (bf16) = silu(gate) up, every
+//     bit as omx_swiglu_forward over C would have it; shapes without that store pass take the pass.
 // aux tensors have C's layout (pitch, and batch stride in a strided batch).
-enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3 };
+enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3, OMX_EPI_SWIGLU = 4 };
 // A term of small rank beside a bf16 product, added in its accumulators (GemmArgs: lr_*).
 struct OmxLowRank {
   const void *h, *w;
@@ -312,6 +314,7 @@ int32_t omx_convert(omx_ctx* ctx, const void* src, int32_t src_dtype, void* dst,
 // ---- device helpers ----
 typedef __hip_bfloat16 bf16_t;
 
+__device__ __forceinline__ float dev_sigmoid(float x) { return 1.0f / (1.0f + __expf(-x)); }
 __device__ __forceinline__ bool dev_finite(float x) {
   return (__float_as_uint(x) & 0x7fffffffu) < 0x7f800000u;
 }

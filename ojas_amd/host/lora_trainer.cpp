@@ -175,8 +175,7 @@ int32_t forward(olora* t) {
     TRY(q8_forward(t, A.ap, A.o, &lr_o, t->t_f));
     TRY(omx_residual_add_rms_norm_forward(ctx, A.x, OMX_F32, t->t_f, OMX_F32, t->norm(l, 1), A.x1, t->h2, OMX_BF16, N, d,
                                           eps));
-    TRY(q8_forward(t, t->h2, A.gu, nullptr, A.gu_out));
-    TRY(omx_swiglu_forward(ctx, A.gu_out, t->m, OMX_F32, N, Hd));
+    TRY(omx_linear_i8_group_swiglu_forward(ctx, t->h2, OMX_BF16, A.gu.codes, A.gu.scales, 32, OMX_I8_BLOCKED, A.gu_out, t->m, N, A.gu.kin, Hd));
     TRY(q8_forward(t, t->m, A.dn, nullptr, t->t_f));
     float* x_next = last ? t->x_final : t->layers[l + 1].x;
     void* h_next = last ? t->hf : t->layers[l + 1].h1;

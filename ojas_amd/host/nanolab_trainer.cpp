@@ -224,8 +224,7 @@ int32_t forward(onano* t) {
     TRY(omx_residual_add_rms_norm_forward(ctx, A.x, OMX_F32, t->t_f, LD, t->w32(t->li(l, NORM2)), A.x1, A.h2, AD, N, d,
                                           eps));
     if (t->fused_mlp) {
-      TRY(omx_linear_forward(ctx, A.h2, AD, t->w(t->li(l, FFN_GATE)), AD, A.gu, LD, N, d, 2 * Hd));
-      TRY(omx_swiglu_forward(ctx, A.gu, A.m, LD, N, Hd));
+      TRY(omx_linear_swiglu_forward(ctx, A.h2, t->w(t->li(l, FFN_GATE)), AD, A.gu, LD, A.m, N, d, Hd));
     } else {
       TRY(omx_linear_forward(ctx, A.h2, AD, t->w(t->li(l, FFN_GATE)), AD, A.g_lin, AD, N, d, Hd));
       TRY(omx_silu_forward(ctx, A.g_lin, A.g_act, AD, N * Hd));

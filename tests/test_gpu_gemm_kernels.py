@@ -794,3 +794,46 @@ def test_products_of_one_launch_are_in_the_profile(be):
     assert launches.value == 1 + 15 and ms.value > 0
     ns = sum(5 * 2.0 * (2 * min(d) ** 2 * max(d) + min(d) ** 3) for d in dims)
     assert flops.value == 4.0 * 1024 * 256 * 128 + ns
+
+
+@pytest.mark.parametrize("rows,kin,hidden,mode", [(300, 128, 64, 9), (256, 256, 192, 9), (1, 384, 128, 9), (513, 128, 320, 9), (300, 128, 72, 9),
+                                                 (300, 192, 64, 1), (70, 64, 8, 1), (8192, 256, 1024, 1), (9000, 128, 1984, 1)])
+def test_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be, rows, kin, hidden, mode):
+    """linear_swiglu_forward, with the activation in the one-wave kernel's store pass (ragged rows, half tiles of units, a product cut by
+    rows) and where it takes the pass: product and activation as linear_forward and swiglu_forward leave them; over int8 codes too; then
+    a gate whose activation is the first value that is not finite."""
+    from ojas_amd.backend import BF16, F32, OjasError, _native
+
+    rng = np.random.default_rng(rows + hidden)
+    x = be.upload(rng.normal(size=(rows, kin)).astype(np.float32), BF16)
+    w = be.upload((0.2 * rng.normal(size=(2 * hidden, kin))).astype(np.float32), BF16)
+    be.set_option("gemm_dma", mode)
+    try:
+        gu = be.linear_forward(x, w, F32)
+        act = be.swiglu_forward(gu)
+        got_gu, got = be.empty((rows, 2 * hidden), F32), be.empty((rows, hidden), BF16)
+        _native.omx_linear_swiglu_forward(be._context, x, w, BF16, got_gu, F32, got, rows, kin, hidden)
+        np.testing.assert_array_equal(be.download(got_gu), be.download(gu))
+        np.testing.assert_array_equal(be.download(got), be.download(act))
+        gu16 = be.linear_forward(x, w, BF16)
+        got16 = be.empty((rows, 2 * hidden), BF16)
+        _native.omx_linear_swiglu_forward(be._context, x, w, BF16, got16, BF16, got, rows, kin, hidden)
+        np.testing.assert_array_equal(be.download(got16), be.download(gu16))
+        np.testing.assert_array_equal(be.download(got), be.download(be.swiglu_forward(gu16)))
+        if kin % 128 == 0:
+            codes, scales = rng.integers(-127, 128, (2 * hidden, kin)).astype(np.int8), rng.uniform(1e-3, 2e-3, (2 * hidden, kin // 32)).astype(np.float32)
+            codes, scales = be.upload(codes), be.upload(scales)
+            for widen in (0, 1):
+                be.set_option("q8_widen", widen)
+                _native.omx_linear_i8_group_forward(be._context, x, BF16, codes, scales, 32, 0, None, None, gu, F32, rows, kin, 2 * hidden)
+                _native.omx_linear_i8_group_swiglu_forward(be._context, x, BF16, codes, scales, 32, 0, got_gu, got, rows, kin, hidden)
+                np.testing.assert_array_equal(be.download(got_gu), be.download(gu))
+                np.testing.assert_array_equal(be.download(got), be.download(be.swiglu_forward(gu)))
+        big = be.upload(np.full((rows, kin), 2.0**60, np.float32), BF16)
+        _native.omx_linear_swiglu_forward(be._context, big, be.upload(np.full((2 * hidden, kin), 2.0**10, np.float32), BF16), BF16, got_gu, F32, got, rows,
+                                          kin, hidden)
+        with pytest.raises(OjasError):
+            be.sync()
+    finally:
+        be.set_option("gemm_dma", 1)
+        be.set_option("q8_widen", -1)
