@@ -593,6 +593,13 @@ int32_t omx_linear_swiglu_forward(omx_ctx* ctx, const void* x, const void* w, in
 int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32,
                                            uint64_t group, int32_t layout, void* gate_up, void* out, uint64_t rows, uint64_t kin,
                                            uint64_t hidden);
+/* omx_linear_i8_group_forward of a fused q | k | v projection (n_out = (heads + plain_heads) dim) into f32 and omx_rope_half_split_pitched of
+ * that, every bit of `out` [rows, n_out] bf16 as those two calls have it. scratch_f32 [rows, n_out] holds the product where it takes two
+ * launches; what it holds afterwards is not defined. */
+int32_t omx_linear_i8_group_rope_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32,
+                                         uint64_t group, int32_t layout, const omx_low_rank* low_rank, void* scratch_f32, void* out,
+                                         const void* cos_f32, const void* sin_f32, uint64_t rows, uint64_t kin, uint64_t time,
+                                         uint64_t heads, uint64_t plain_heads, uint64_t dim);
 /* Synthetic weights made on the device (no counterpart in the reference, whose init runs on the
  * host, ojas-model/src/init.rs:67-114): element i is N(0, std) from a counter-based generator of
  * (seed, i). omx_init_normal_i8_group draws row-major [n_out, k_in] values and stores them

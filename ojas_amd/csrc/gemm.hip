@@ -593,7 +593,16 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   const OmxGemmEpilogue* swiglu = epi && epi->mode == OMX_EPI_SWIGLU ? epi : nullptr;
   if (swiglu && (operand_dtype != OMX_BF16 || c_dtype != OMX_F32 || accumulate || batches != 1 || low_rank || ldc != n || n % 2 != 0))
     return omx_fail(ctx, OMX_UNSUPPORTED, "%s: gates and ups go with one plain bf16 product into f32", op);
-  if (sum32 || act32 || swiglu) epi = nullptr;
+  // Heads that turn (OMX_EPI_ROPE): likewise, beside a low-rank term.
+  const OmxGemmEpilogue* rope = epi && epi->mode == OMX_EPI_ROPE ? epi : nullptr;
+  if (rope && (operand_dtype != OMX_BF16 || c_dtype != OMX_F32 || accumulate || batches != 1 || ldc != n))
+    return omx_fail(ctx, OMX_UNSUPPORTED, "%s: heads turn behind one plain bf16 product into f32", op);
+  auto turn = [&]() {
+    return omx_rope_half_split_pitched(ctx, c, OMX_F32, rope->aux_out, n, rope->rope.cos_t, rope->rope.sin_t, m, static_cast<uint64_t>(rope->rope.time),
+                                       static_cast<uint64_t>(rope->rope.heads), static_cast<uint64_t>(rope->rope.plain),
+                                       static_cast<uint64_t>(rope->rope.dim));
+  };
+  if (sum32 || act32 || swiglu || rope) epi = nullptr;
   if (epi && epi->mode != OMX_EPI_NONE && c_dtype != OMX_BF16)
     return omx_fail(ctx, OMX_DTYPE, "%s: a fused activation needs a bf16 output", op);
   if (!a || !b || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
@@ -822,7 +831,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
                            operand_dtype, static_cast<char*>(c) + m0 * ldc * csz, c_dtype, ldc, m - m0, k, n,
                            accumulate, swiglu ? &rest_pairs : epi, nullptr, a_k, low_rank ? &rest_rank : nullptr);
       ctx->gemm_in_row_split = false;
-      return rc;
+      return rc == OMX_OK && rope ? turn() : rc;
     }
   }
   int BM = 128, BN = 128;
@@ -937,7 +946,15 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   }
   g.fault = ctx->fault;
   g.tag = omx_tag(ctx, fault_op);
-  if (pairs_fused) g.act_tag = omx_tag(ctx, F_MUL_FORWARD);
+  const bool rope_fused = rope && dma_variant == 9 && !a_km && !b_km && g.splits == 1 && g.lr_rank > 0 && n % 128 == 0 && g.c_vec &&
+                          (rope->rope.dim == 64 || rope->rope.dim == 128) && rope->rope.heads * rope->rope.dim % 128 == 0 &&
+                          aligned16(rope->aux_out) && aligned16(rope->rope.cos_t) && aligned16(rope->rope.sin_t);
+  if (rope_fused) {
+    g.epi = OMX_EPI_ROPE;
+    g.rope = rope->rope;
+    g.aux_out = static_cast<unsigned short*>(rope->aux_out);
+  }
+  if (pairs_fused || rope_fused) g.act_tag = omx_tag(ctx, pairs_fused ? F_MUL_FORWARD : F_ROPE_FORWARD);
   else g.act_tag = act_fused ? omx_tag(ctx, act32->mode == OMX_EPI_GELU_FWD ? F_GELU_FORWARD : F_GELU_BACKWARD) : g.tag;
   omx_ctx::TimedLaunch timed{};
   if (ctx->profile_gemm) {
@@ -983,6 +1000,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     ctx->timing_start = ctx->timing_stop = nullptr;
     if (rc == OMX_OK) ctx->timed.push_back(timed);
   }
+  if (rc == OMX_OK && rope && !rope_fused) rc = turn();
   if (rc == OMX_OK && swiglu && !pairs_fused) rc = omx_swiglu_forward(ctx, c, swiglu->aux_out, OMX_F32, m, n / 2);
   if (rc == OMX_OK && act32 && !act_fused)
     rc = act32->mode == OMX_EPI_GELU_FWD ? omx_gelu_forward(ctx, c, act32->aux_out, OMX_F32, m * n, act32->tanh_form)

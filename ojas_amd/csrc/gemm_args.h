@@ -28,6 +28,7 @@ struct GemmArgs {
   const unsigned short *lr_h, *lr_w;
   long lr_pitch, lr_w_pitch;
   int lr_rank, lr_block_cols;
+  OmxRope rope;  // OMX_EPI_ROPE
   // Strided batch: block (x, y) works on product y, whose operands start batch_* BYTES after
   // product y - 1's. batches == 1 for a single product.
   int batches;

@@ -535,10 +535,10 @@ int32_t widened_product(omx_ctx* ctx, uint32_t fault_op, const Q8Args& g, uint64
   return *taken ? rc : OMX_OK;
 }
 
-// `swiglu`: the products' columns are gates and ups, and their activation goes there (OMX_EPI_SWIGLU).
+// `after`: OMX_EPI_SWIGLU or OMX_EPI_ROPE of the product.
 int32_t i8_forward(omx_ctx* ctx, const char* op, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32, uint64_t group,
                    int32_t layout, const void* add, const omx_low_rank* low_rank, void* y, int32_t y_dtype, uint64_t rows, uint64_t kin,
-                   uint64_t nout, void* swiglu) {
+                   uint64_t nout, const OmxGemmEpilogue* after) {
   int32_t rc = check_q8(ctx, op, x, codes_i8, scales_f32, y, add, rows, kin, nout, group, x_dtype, layout);
   if (rc != OMX_OK) return rc;
   if (!omx_valid_float_dtype(y_dtype)) return omx_fail(ctx, OMX_DTYPE, "%s: the output must be f32 or bf16", op);
@@ -563,12 +563,16 @@ int32_t i8_forward(omx_ctx* ctx, const char* op, const void* x, int32_t x_dtype,
   rc = set_low_rank(ctx, op, &g, low_rank, nout);
   if (rc != OMX_OK) return rc;
   bool taken = false;
-  const OmxGemmEpilogue pairs = {OMX_EPI_SWIGLU, 0, nullptr, swiglu};
-  rc = widened_product(ctx, F_LINEAR_FORWARD, g, rows, kin, nout, false, &taken, swiglu ? &pairs : nullptr);
+  rc = widened_product(ctx, F_LINEAR_FORWARD, g, rows, kin, nout, false, &taken, after);
   if (rc != OMX_OK || taken) return rc;
   g.tag = omx_tag(ctx, F_LINEAR_FORWARD);
   rc = launch_q8<false>(ctx, g, 2.0 * rows * kin * nout);
-  return rc == OMX_OK && swiglu ? omx_swiglu_forward(ctx, y, swiglu, OMX_F32, rows, nout / 2) : rc;
+  if (rc != OMX_OK || !after) return rc;
+  const OmxRope& turn = after->rope;
+  return after->mode == OMX_EPI_SWIGLU
+             ? omx_swiglu_forward(ctx, y, after->aux_out, OMX_F32, rows, nout / 2)
+             : omx_rope_half_split_pitched(ctx, y, OMX_F32, after->aux_out, nout, turn.cos_t, turn.sin_t, rows, static_cast<uint64_t>(turn.time),
+                                           static_cast<uint64_t>(turn.heads), static_cast<uint64_t>(turn.plain), static_cast<uint64_t>(turn.dim));
 }
 
 }  // namespace
@@ -588,7 +592,25 @@ int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t 
   OMX_REQUIRE_CTX(ctx);
   const char* op = "linear_i8_group_swiglu_forward";
   if (!out) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
-  return i8_forward(ctx, op, x, x_dtype, codes_i8, scales_f32, group, layout, nullptr, nullptr, gate_up, OMX_F32, rows, kin, 2 * hidden, out);
+  const OmxGemmEpilogue pairs = {OMX_EPI_SWIGLU, 0, nullptr, out};
+  return i8_forward(ctx, op, x, x_dtype, codes_i8, scales_f32, group, layout, nullptr, nullptr, gate_up, OMX_F32, rows, kin, 2 * hidden, &pairs);
+}
+
+int32_t omx_linear_i8_group_rope_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32, uint64_t group,
+                                         int32_t layout, const omx_low_rank* low_rank, void* scratch_f32, void* out, const void* cos_f32,
+                                         const void* sin_f32, uint64_t rows, uint64_t kin, uint64_t time, uint64_t heads, uint64_t plain_heads,
+                                         uint64_t dim) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "linear_i8_group_rope_forward";
+  if (!out || !cos_f32 || !sin_f32) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (time == 0 || dim == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
+  if (time > 0x7fffffffull || dim > 0x7fffffffull || heads > 0x7fffffffull || plain_heads > 0x7fffffffull || (heads + plain_heads) * dim > 0x7fffffffull)
+    return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: axis does not fit in i32", op);
+  OmxGemmEpilogue turn = {OMX_EPI_ROPE, 0, nullptr, out};
+  turn.rope = {static_cast<const float*>(cos_f32), static_cast<const float*>(sin_f32), static_cast<int>(time), static_cast<int>(heads),
+               static_cast<int>(plain_heads), static_cast<int>(dim)};
+  return i8_forward(ctx, op, x, x_dtype, codes_i8, scales_f32, group, layout, nullptr, low_rank, scratch_f32, OMX_F32, rows, kin,
+                    (heads + plain_heads) * dim, &turn);
 }
 
 int32_t omx_linear_i8_group_backward_input(omx_ctx* ctx, const void* codes_i8, const void* scales_f32, uint64_t group,

@@ -132,14 +132,19 @@ struct W4Frags {
 };
 
 // LR: with a low-rank term.
+// STORE: OMX_EPI_SWIGLU and OMX_EPI_ROPE have a store pass of their own.
 // PAIR: B's rows are gates and, N / 2 further, ups. A wave's 128 columns are 64 units' gates and ups, which meet in its store pass: C
 // as it would be, in f32, and silu(gate) up beside it in bf16 (OMX_EPI_SWIGLU), where a pass of its own read C again. us, product and pass / so,
 // inside a step: 8192 rows over 2048 -> 2 x 8192: 490 + 112 / 545; 16384 over 768 -> 2 x 2048: 130 + 59 / 154.
-template <bool A_KM, bool B_KM, int TN, bool TAIL, bool LR = false, bool PAIR = false>
+// ROPE: heads of 64 or 128 columns are turned in the store pass (OMX_EPI_ROPE), where the product went out in f32 and a pass read it: both halves of a
+// head lie in a wave's 128 columns. us, product and pass / so, inside a step: 8192 rows over
+// 2048 -> 48 heads of 128, two thirds of them turned: 213 + 51 / 204 (tables read row by row, after the staging: 241).
+template <bool A_KM, bool B_KM, int TN, bool TAIL, bool LR = false, int STORE = OMX_EPI_NONE>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   static_assert(!A_KM || B_KM, "a k-major A goes with a k-major B");
   static_assert(TN == 4 || TN == 3, "256 x 256 or 256 x 192 tiles");
-  static_assert(!PAIR || (!A_KM && !B_KM && TN == 4 && !TAIL && !LR), "one form of pairs");
+  constexpr bool PAIR = STORE == OMX_EPI_SWIGLU, ROPE = STORE == OMX_EPI_ROPE;
+  static_assert(!(PAIR || ROPE) || (!A_KM && !B_KM && TN == 4 && !TAIL && LR == ROPE), "one form of each");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr int TM = 4, NW = 4, W4_BN = TN * 64;
   // Tile order: as gemm_dma_kernel.
@@ -461,7 +466,58 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
     constexpr int tm = decltype(tm_index)::value;
     const int grow0 = m0 + (wm * TM + tm) * 32;
     const bool interior = grow0 + 32 <= g.M && gcol0 + TN * 32 <= g.N;
-    if constexpr (PAIR) {
+    if constexpr (ROPE) {
+      const int dim = g.rope.dim, per = dim / 8, head = (lane & 15) / per, at = (lane & 15) % per * 4, lo = head * dim + at;
+      const bool turn = gcol0 < g.rope.heads * dim;  // (N and the columns that turn are multiples of 128)
+      float4 c4[8], s4[8];  // on their way while the rows are staged
+      if (turn) {
+        int t = (grow0 + (lane >> 4)) % g.rope.time;
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+          const long from = static_cast<long>(t) * dim + at;
+          c4[it] = *reinterpret_cast<const float4*>(g.rope.cos_t + from);
+          s4[it] = *reinterpret_cast<const float4*>(g.rope.sin_t + from);
+          t += 4;
+          while (t >= g.rope.time) t -= g.rope.time;
+        }
+      }
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const floatx16& c = acc[tm][tn];
+          *reinterpret_cast<float4*>(cs + l32 * CPW + tn * 32 + 8 * q + 4 * lg) = make_float4(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]);
+        }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (gcol0 < g.N) {
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+          const int row = it * 4 + (lane >> 4);
+          const float4 x = *reinterpret_cast<const float4*>(cs + row * CPW + lo), y = *reinterpret_cast<const float4*>(cs + row * CPW + lo + dim / 2);
+          const float a[4] = {x.x, x.y, x.z, x.w}, b[4] = {y.x, y.y, y.z, y.w};
+          float ya[4] = {x.x, x.y, x.z, x.w}, yb[4] = {y.x, y.y, y.z, y.w};
+          if (turn) {
+            const float c[4] = {c4[it].x, c4[it].y, c4[it].z, c4[it].w}, s[4] = {s4[it].x, s4[it].y, s4[it].z, s4[it].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              ya[e] = a[e] * c[e] - b[e] * s[e];
+              yb[e] = b[e] * c[e] + a[e] * s[e];
+            }
+          }
+          if (grow0 + row < g.M) {
+            unsigned short* to = g.aux_out + static_cast<long>(grow0 + row) * g.ldc + gcol0 + lo;
+            *reinterpret_cast<uint2*>(to) = make_uint2(dev_pack_bf16_pair(ya[0], ya[1]), dev_pack_bf16_pair(ya[2], ya[3]));
+            *reinterpret_cast<uint2*>(to + dim / 2) = make_uint2(dev_pack_bf16_pair(yb[0], yb[1]), dev_pack_bf16_pair(yb[2], yb[3]));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              bad |= !(dev_finite(a[e]) && dev_finite(b[e]));
+              bad_act |= !(dev_finite(ya[e]) && dev_finite(yb[e]));
+            }
+          }
+        }
+      }
+    } else if constexpr (PAIR) {
       const int half = g.N / 2, unit0 = n0 / 2 + wn * 64;
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn)
@@ -551,7 +607,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   });
   bad |= (flags & 0x80008000u) != 0;
   if (bad) dev_raise_fault(g.fault, g.tag);
-  if (PAIR && bad_act && !bad) dev_raise_fault(g.fault, g.act_tag);
+  if (STORE && bad_act && !bad) dev_raise_fault(g.fault, g.act_tag);
 }
 
 template <bool A_KM, bool B_KM, int TN>
@@ -564,7 +620,8 @@ int32_t launch_w4(omx_ctx* ctx, const GemmArgs& g) {
     if (g.lr_rank > 0) kernel = &gemm_w4_kernel<A_KM, B_KM, TN, false, true>;  // (whole steps)
   }
   if constexpr (!A_KM && !B_KM && TN == 4) {
-    if (g.epi == OMX_EPI_SWIGLU) kernel = &gemm_w4_kernel<false, false, 4, false, false, true>;
+    if (g.epi == OMX_EPI_SWIGLU) kernel = &gemm_w4_kernel<false, false, 4, false, false, OMX_EPI_SWIGLU>;
+    if (g.epi == OMX_EPI_ROPE) kernel = &gemm_w4_kernel<false, false, 4, false, true, OMX_EPI_ROPE>;
   }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    W4_SMEM));

@@ -238,8 +238,15 @@ inline unsigned long long omx_tag(omx_ctx* ctx, uint32_t op) {
 //     s2 A.B, each term rounded as a pass of its own would.
 //   OMX_EPI_SWIGLU: C (f32, its first half of columns gates, the second ups) = A.B and aux_out [m, n / 2] (bf16) = silu(gate) up, every
 //     bit as omx_swiglu_forward over C would have it; shapes without that store pass take the pass.
+//   OMX_EPI_ROPE: aux_out [m, n] (bf16) = what omx_rope_half_split_pitched makes of A.B in f32, its bits; C (f32, [m, n]) is scratch for shapes
+//     that take the pass, and is left alone otherwise.
 // aux tensors have C's layout (pitch, and batch stride in a strided batch).
-enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3, OMX_EPI_SWIGLU = 4 };
+enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3, OMX_EPI_SWIGLU = 4, OMX_EPI_ROPE = 5 };
+// The rotation of OMX_EPI_ROPE: tables [time, dim], rows are tokens of sequences of `time`, the first `heads` heads turn, `plain` follow.
+struct OmxRope {
+  const float *cos_t, *sin_t;
+  int time, heads, plain, dim;
+};
 // A term of small rank beside a bf16 product, added in its accumulators (GemmArgs: lr_*).
 struct OmxLowRank {
   const void *h, *w;
@@ -251,6 +258,7 @@ struct OmxGemmEpilogue {
   const void* aux_in;
   void* aux_out;
   float s1 = 0.0f, s2 = 0.0f;  // OMX_EPI_AXPBY
+  OmxRope rope = {};           // OMX_EPI_ROPE
 };
 // `count` products of one shape whose operands lie `stride_*` ELEMENTS apart (16-byte multiples), one launch.
 struct OmxGemmBatch {

@@ -164,8 +164,8 @@ int32_t forward(olora* t) {
     // h A^T for the three sites at once: [N, 3r] in the first columns of ha.
     TRY(omx_gemm_pitched(ctx, A.h1, d, 1, t->a16(l, 0), 1, d, OMX_BF16, A.ha, OMX_BF16, 4 * r, N, d, 3 * r, 0));
     omx_low_rank lr_qkv{A.ha, t->b16(l, 0), 4 * r, r, r, d};
-    TRY(q8_forward(t, A.h1, A.qkv, &lr_qkv, t->qkv32));
-    TRY(omx_rope_half_split_pitched(ctx, t->qkv32, OMX_F32, A.qkv_out, 3 * d, t->cos_t, t->sin_t, N, T, 2 * H, H, D));
+    TRY(omx_linear_i8_group_rope_forward(ctx, A.h1, OMX_BF16, A.qkv.codes, A.qkv.scales, 32, OMX_I8_BLOCKED, &lr_qkv, t->qkv32, A.qkv_out,
+                                         t->cos_t, t->sin_t, N, A.qkv.kin, T, 2 * H, H, D));
     // The output's rounding residual is kept for the backward's row term, as the reference keeps
     // its saved output unrounded (ojas-core/src/autocast.rs:177-186).
     TRY(omx_causal_attention_forward_saving(ctx, A.qkv_out, 3 * d, off16(A.qkv_out, d), off16(A.qkv_out, 2 * d), 3 * d,

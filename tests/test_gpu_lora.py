@@ -200,6 +200,43 @@ def test_blocked_layout_gives_the_same_products(be, rows, kin, nout):
         assert np.array_equal(g0, g1)
 
 
+@pytest.mark.parametrize("rows,kin,time,heads,plain,dim,mode", [(300, 128, 70, 4, 2, 64, 9), (257, 256, 257, 2, 1, 128, 9), (513, 128, 3, 2, 3, 128, 9),
+                                                               (40, 128, 1, 2, 2, 64, 9), (300, 128, 100, 2, 1, 64, 9), (300, 128, 100, 2, 1, 32, 9),
+                                                               (300, 256, 150, 4, 2, 64, 1), (8192, 256, 512, 8, 4, 128, 1)])
+@pytest.mark.parametrize("ranked", [True, False])
+def test_turned_heads_of_one_product_have_the_bits_of_two_calls(be, rows, kin, time, heads, plain, dim, mode, ranked):
+    """linear_i8_group_rope_forward, with the rotation in the one-wave kernel's store pass (both head widths, ragged rows, sequences that end
+    inside a row block) and where it takes the pass, over the codes and over a widened copy; then a product that is not finite."""
+    from ojas_amd.backend import BF16, F32, OjasError, _native
+
+    nout, rank = (heads + plain) * dim, 16
+    rng = np.random.default_rng(rows + nout)
+    x = be.upload(rng.normal(size=(rows, kin)).astype(np.float32), BF16)
+    codes = be.upload(rng.integers(-127, 128, (nout, kin)).astype(np.int8))
+    scales = be.upload(rng.uniform(1e-3, 2e-3, (nout, kin // 32)).astype(np.float32))
+    cos, sin = (be.upload(f(np.outer(np.arange(time), rng.uniform(0.01, 1.0, dim))).astype(np.float32)) for f in (np.cos, np.sin))
+    low_rank = (be.upload(rng.normal(size=(rows, rank)).astype(np.float32), BF16),
+                be.upload(rng.normal(size=(nout, rank)).astype(np.float32), BF16), 0) if ranked else None
+    tail, tail_at = be._low_rank(low_rank)
+    be.set_option("gemm_dma", mode)
+    try:
+        for widen in (0, 1):
+            be.set_option("q8_widen", widen)
+            y = be.linear_i8_group_forward(x, codes, scales, low_rank=low_rank, out_dtype=F32)
+            want, got, scratch = be.empty((rows, nout), BF16), be.empty((rows, nout), BF16), be.empty((rows, nout), F32)
+            _native.omx_rope_half_split_pitched(be._context, y, F32, want, nout, cos, sin, rows, time, heads, plain, dim)
+            call = lambda a, s: _native.omx_linear_i8_group_rope_forward(be._context, a, BF16, codes, s, 32, 0, tail_at, scratch, got, cos, sin, rows, kin, time,
+                                                                         heads, plain, dim)
+            call(x, scales)
+            np.testing.assert_array_equal(be.download(got), be.download(want))
+        call(be.upload(np.full((rows, kin), 2.0**100, np.float32), BF16), be.upload(np.full((nout, kin // 32), 2.0**30, np.float32)))
+        with pytest.raises(OjasError):
+            be.sync()
+    finally:
+        be.set_option("gemm_dma", 1)
+        be.set_option("q8_widen", -1)
+
+
 @pytest.mark.parametrize("rows,kin,nout,rank,blocks", [(300, 128, 256, 16, 1), (520, 256, 384, 16, 3),
                                                          (256, 64, 128, 48, 1)])
 def test_low_rank_term_rides_in_the_accumulators(be, rows, kin, nout, rank, blocks):
