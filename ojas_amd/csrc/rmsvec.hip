@@ -428,9 +428,16 @@ int32_t omx_rms_forward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const 
 int32_t omx_rms_backward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const float* w, const void* gy,
                              int32_t gy_dtype, const float* add_in, void* gx, int32_t gx_dtype, void* gx16, float* gw,
                              uint64_t rows, uint64_t dim, float eps, unsigned long long tag) {
-  // The kernel's time does not depend on the rows a block takes between 2 and 16 per wave (the
-  // loads of a row are all in flight at once); fewer blocks leave fewer partial rows to add.
-  int rows_per_block = 8;
+  // A wave's rows are a chain of two reductions each, all its time where rows are few: a row a wave then, while that leaves
+  // no more partial rows than their sum takes for nothing (us at 8 rows a block and at 4, gradient of the weight with its
+  // sum: 169 x 1152 11.8 to 8.6, 516 x 640 7.6 to 6.9, 1024 x 768 7.9 and 7.8; up to 192 partial rows its error against f64
+  // is as at 8 rows, 1.12e-7 of its size at 516 x 640 where that has 1.18e-7; at 512 partial rows it is 3 % above). A frozen
+  // weight has no partial rows, and fewer rows than compute units take one each (169 x 1152: 7.6 at 8 rows, 5.0 at 4, 4.5
+  // at 1; 256 x 2048 9.3, 5.5, 5.0; 2048 x 2048 14.4, 12.4). Over many rows the time does not depend on the rows a block
+  // takes between 2 and 16 per wave, and fewer blocks leave fewer partial rows to add.
+  const bool few = rows <= 768 && omx_workspace_fits(ctx, ((rows + 3) / 4 + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float));
+  int rows_per_block = !gw || few ? 4 : 8;
+  if (!gw && rows <= static_cast<uint64_t>(ctx->cu_count)) rows_per_block = 1;
   while (rows_per_block < (dim > 1024 ? 16 : 32) && rows / rows_per_block > 512) rows_per_block *= 2;
   const uint64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
   // A null gw: the weight is frozen, its gradient is not formed (no partial sums, no second launch).

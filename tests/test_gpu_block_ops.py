@@ -440,7 +440,7 @@ def test_gate_backward_without_its_weight_gradient(be, rows, d_model, heads, hea
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("rows,dim", [(5, 256), (33, 768), (1000, 768), (17, 1024), (9, 260), (40, 96), (12, 2048),
                                       (33, 1284), (70, 2044), (9000, 768), (40000, 512), (5000, 2048),
-                                      (2048, 768), (2049, 768)])
+                                      (2048, 768), (2049, 768), (256, 1028), (257, 1028), (767, 640), (769, 640)])
 def test_fused_residual_rms_norm_equals_the_separate_ops(be, rows, dim, bf16):
     """block.rs:247-249 (add, then norm) and the tape's fan-in at a residual: the fused entry points
     must give the bits of the separate calls, and the norm itself must match the oracle. The
