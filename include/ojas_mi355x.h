@@ -593,6 +593,15 @@ int32_t omx_linear_swiglu_forward(omx_ctx* ctx, const void* x, const void* w, in
 int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32,
                                            uint64_t group, int32_t layout, void* gate_up, void* out, uint64_t rows, uint64_t kin,
                                            uint64_t hidden);
+/* The input gradient of linear_backward (backend.rs:1628-1645) of the projection behind a SwiGLU, w [out, hidden] bf16, and swiglu_backward of
+ * it: every bit of g_gate_up [rows, 2 hidden] bf16 as those two calls have it. scratch [rows, hidden] bf16 holds the product where it takes
+ * two launches; what it holds afterwards is not defined. The second form over int8 codes (omx_linear_i8_group_backward_input, gate_up f32). */
+int32_t omx_linear_backward_input_swiglu(omx_ctx* ctx, const void* w, const void* gy, int32_t operand_dtype, const void* gate_up,
+                                         int32_t gate_up_dtype, void* scratch, void* g_gate_up, uint64_t rows, uint64_t hidden,
+                                         uint64_t out_features);
+int32_t omx_linear_i8_group_backward_input_swiglu(omx_ctx* ctx, const void* codes_i8, const void* scales_f32, uint64_t group, int32_t layout,
+                                                  const void* gy, int32_t gy_dtype, const void* gate_up, void* scratch, void* g_gate_up,
+                                                  uint64_t rows, uint64_t hidden, uint64_t nout);
 /* omx_linear_i8_group_forward of a fused q | k | v projection (n_out = (heads + plain_heads) dim) into f32 and omx_rope_half_split_pitched of
  * that, every bit of `out` [rows, n_out] bf16 as those two calls have it. scratch_f32 [rows, n_out] holds the product where it takes two
  * launches; what it holds afterwards is not defined. */

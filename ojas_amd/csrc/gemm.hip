@@ -602,7 +602,11 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
                                        static_cast<uint64_t>(rope->rope.heads), static_cast<uint64_t>(rope->rope.plain),
                                        static_cast<uint64_t>(rope->rope.dim));
   };
-  if (sum32 || act32 || swiglu || rope) epi = nullptr;
+  // The gradients of gates and ups (OMX_EPI_SWIGLU_BWD): likewise, the product being that of silu(gate) up.
+  const OmxGemmEpilogue* dswiglu = epi && epi->mode == OMX_EPI_SWIGLU_BWD ? epi : nullptr;
+  if (dswiglu && (operand_dtype != OMX_BF16 || c_dtype != OMX_BF16 || accumulate || batches != 1 || low_rank || ldc != n))
+    return omx_fail(ctx, OMX_UNSUPPORTED, "%s: gradients of gates and ups go with one plain bf16 product", op);
+  if (sum32 || act32 || swiglu || rope || dswiglu) epi = nullptr;
   if (epi && epi->mode != OMX_EPI_NONE && c_dtype != OMX_BF16)
     return omx_fail(ctx, OMX_DTYPE, "%s: a fused activation needs a bf16 output", op);
   if (!a || !b || !c) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
@@ -814,7 +818,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
       ctx->gemm_in_row_split = true;
       ctx->gemm_forced_tiling = dma_variant;
       int32_t rc = omx_gemm_impl(ctx, fault_op, a, a_rs, a_cs, b, b_rs, b_cs, operand_dtype, c, c_dtype, ldc, m0, k, n,
-                                 accumulate, swiglu ? swiglu : epi, nullptr, a_k, low_rank);
+                                 accumulate, swiglu ? swiglu : dswiglu ? dswiglu : epi, nullptr, a_k, low_rank);
       ctx->gemm_forced_tiling = -1;
       OmxLowRank rest_rank{};
       if (low_rank) {
@@ -826,10 +830,15 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
         rest_pairs = *swiglu;
         rest_pairs.aux_out = static_cast<unsigned short*>(swiglu->aux_out) + m0 * (n / 2);
       }
+      if (dswiglu) {
+        rest_pairs = *dswiglu;
+        rest_pairs.aux_in = static_cast<const float*>(dswiglu->aux_in) + m0 * 2 * n;
+        rest_pairs.aux_out = static_cast<unsigned short*>(dswiglu->aux_out) + m0 * 2 * n;
+      }
       if (rc == OMX_OK)
         rc = omx_gemm_impl(ctx, fault_op, static_cast<const char*>(a) + m0 * a_rs * esz, a_rs, a_cs, b, b_rs, b_cs,
                            operand_dtype, static_cast<char*>(c) + m0 * ldc * csz, c_dtype, ldc, m - m0, k, n,
-                           accumulate, swiglu ? &rest_pairs : epi, nullptr, a_k, low_rank ? &rest_rank : nullptr);
+                           accumulate, swiglu || dswiglu ? &rest_pairs : epi, nullptr, a_k, low_rank ? &rest_rank : nullptr);
       ctx->gemm_in_row_split = false;
       return rc == OMX_OK && rope ? turn() : rc;
     }
@@ -954,7 +963,15 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     g.rope = rope->rope;
     g.aux_out = static_cast<unsigned short*>(rope->aux_out);
   }
-  if (pairs_fused || rope_fused) g.act_tag = omx_tag(ctx, pairs_fused ? F_MUL_FORWARD : F_ROPE_FORWARD);
+  const bool dpairs_fused = dswiglu && dma_variant == 9 && !a_km && b_km && g.splits == 1 && g.k_rows == g.K && n % 128 == 0 &&
+                            aligned16(dswiglu->aux_in) && aligned16(dswiglu->aux_out);
+  if (dpairs_fused) {
+    g.epi = OMX_EPI_SWIGLU_BWD;
+    g.aux_in = static_cast<const unsigned short*>(dswiglu->aux_in);
+    g.aux_out = static_cast<unsigned short*>(dswiglu->aux_out);
+  }
+  if (pairs_fused || rope_fused || dpairs_fused)
+    g.act_tag = omx_tag(ctx, pairs_fused ? F_MUL_FORWARD : rope_fused ? F_ROPE_FORWARD : F_MUL_BACKWARD);
   else g.act_tag = act_fused ? omx_tag(ctx, act32->mode == OMX_EPI_GELU_FWD ? F_GELU_FORWARD : F_GELU_BACKWARD) : g.tag;
   omx_ctx::TimedLaunch timed{};
   if (ctx->profile_gemm) {
@@ -1001,6 +1018,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     if (rc == OMX_OK) ctx->timed.push_back(timed);
   }
   if (rc == OMX_OK && rope && !rope_fused) rc = turn();
+  if (rc == OMX_OK && dswiglu && !dpairs_fused) rc = omx_swiglu_backward(ctx, dswiglu->aux_in, c, dswiglu->aux_out, OMX_F32, m, n);
   if (rc == OMX_OK && swiglu && !pairs_fused) rc = omx_swiglu_forward(ctx, c, swiglu->aux_out, OMX_F32, m, n / 2);
   if (rc == OMX_OK && act32 && !act_fused)
     rc = act32->mode == OMX_EPI_GELU_FWD ? omx_gelu_forward(ctx, c, act32->aux_out, OMX_F32, m * n, act32->tanh_form)

@@ -575,6 +575,40 @@ int32_t i8_forward(omx_ctx* ctx, const char* op, const void* x, int32_t x_dtype,
                                            static_cast<uint64_t>(turn.heads), static_cast<uint64_t>(turn.plain), static_cast<uint64_t>(turn.dim));
 }
 
+// `after`: OMX_EPI_SWIGLU_BWD of the product.
+int32_t i8_backward_input(omx_ctx* ctx, const char* op, const void* codes_i8, const void* scales_f32, uint64_t group, int32_t layout, const void* gy,
+                          int32_t gy_dtype, const void* add, const omx_low_rank* low_rank, void* gx, uint64_t rows, uint64_t kin, uint64_t nout,
+                          const OmxGemmEpilogue* after) {
+  int32_t rc = check_q8(ctx, op, gy, codes_i8, scales_f32, gx, add, rows, kin, nout, group, gy_dtype, layout);
+  if (rc != OMX_OK) return rc;
+  if (nout % 32 != 0)
+    return omx_fail(ctx, OMX_SHAPE, "%s: n_out %llu is not a multiple of 32", op, (unsigned long long)nout);
+  Q8Args g{};
+  g.a = static_cast<const unsigned short*>(gy);
+  g.lda = static_cast<long>(nout);
+  g.codes = static_cast<const signed char*>(codes_i8);
+  g.scales = static_cast<const float*>(scales_f32);
+  g.kin = static_cast<long>(kin);
+  g.c = static_cast<unsigned short*>(gx);
+  g.ldc = static_cast<long>(kin);
+  g.add = static_cast<const unsigned short*>(add);
+  g.M = static_cast<int>(rows);
+  g.N = static_cast<int>(kin);
+  g.K = static_cast<int>(nout);
+  g.tiles_m = (g.M + QBM - 1) / QBM;
+  g.tiles_n = (g.N + QBN - 1) / QBN;
+  g.packed = layout == OMX_I8_BLOCKED;
+  g.fault = ctx->fault;
+  rc = set_low_rank(ctx, op, &g, low_rank, kin);
+  if (rc != OMX_OK) return rc;
+  bool taken = false;
+  rc = widened_product(ctx, F_LINEAR_BACKWARD, g, rows, kin, nout, true, &taken, after);
+  if (rc != OMX_OK || taken) return rc;
+  g.tag = omx_tag(ctx, F_LINEAR_BACKWARD);
+  rc = launch_q8<true>(ctx, g, 2.0 * rows * kin * nout);
+  return rc != OMX_OK || !after ? rc : omx_swiglu_backward(ctx, after->aux_in, gx, after->aux_out, OMX_F32, rows, kin);
+}
+
 }  // namespace
 
 extern "C" {
@@ -618,34 +652,18 @@ int32_t omx_linear_i8_group_backward_input(omx_ctx* ctx, const void* codes_i8, c
                                            const omx_low_rank* low_rank, void* gx, uint64_t rows, uint64_t kin,
                                            uint64_t nout) {
   OMX_REQUIRE_CTX(ctx);
-  const char* op = "linear_i8_group_backward_input";
-  int32_t rc = check_q8(ctx, op, gy, codes_i8, scales_f32, gx, add, rows, kin, nout, group, gy_dtype, layout);
-  if (rc != OMX_OK) return rc;
-  if (nout % 32 != 0)
-    return omx_fail(ctx, OMX_SHAPE, "%s: n_out %llu is not a multiple of 32", op, (unsigned long long)nout);
-  Q8Args g{};
-  g.a = static_cast<const unsigned short*>(gy);
-  g.lda = static_cast<long>(nout);
-  g.codes = static_cast<const signed char*>(codes_i8);
-  g.scales = static_cast<const float*>(scales_f32);
-  g.kin = static_cast<long>(kin);
-  g.c = static_cast<unsigned short*>(gx);
-  g.ldc = static_cast<long>(kin);
-  g.add = static_cast<const unsigned short*>(add);
-  g.M = static_cast<int>(rows);
-  g.N = static_cast<int>(kin);
-  g.K = static_cast<int>(nout);
-  g.tiles_m = (g.M + QBM - 1) / QBM;
-  g.tiles_n = (g.N + QBN - 1) / QBN;
-  g.packed = layout == OMX_I8_BLOCKED;
-  g.fault = ctx->fault;
-  rc = set_low_rank(ctx, op, &g, low_rank, kin);
-  if (rc != OMX_OK) return rc;
-  bool taken = false;
-  rc = widened_product(ctx, F_LINEAR_BACKWARD, g, rows, kin, nout, true, &taken);
-  if (rc != OMX_OK || taken) return rc;
-  g.tag = omx_tag(ctx, F_LINEAR_BACKWARD);
-  return launch_q8<true>(ctx, g, 2.0 * rows * kin * nout);
+  return i8_backward_input(ctx, "linear_i8_group_backward_input", codes_i8, scales_f32, group, layout, gy, gy_dtype, add, low_rank, gx, rows, kin, nout,
+                           nullptr);
+}
+
+int32_t omx_linear_i8_group_backward_input_swiglu(omx_ctx* ctx, const void* codes_i8, const void* scales_f32, uint64_t group, int32_t layout,
+                                                  const void* gy, int32_t gy_dtype, const void* gate_up, void* scratch, void* g_gate_up,
+                                                  uint64_t rows, uint64_t hidden, uint64_t nout) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "linear_i8_group_backward_input_swiglu";
+  if (!gate_up || !g_gate_up) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  const OmxGemmEpilogue pairs = {OMX_EPI_SWIGLU_BWD, 0, gate_up, g_gate_up};
+  return i8_backward_input(ctx, op, codes_i8, scales_f32, group, layout, gy, gy_dtype, nullptr, nullptr, scratch, rows, hidden, nout, &pairs);
 }
 
 int32_t omx_pack_i8_group(omx_ctx* ctx, const void* codes_i8, const void* scales_f32, void* blocked_codes,

@@ -132,19 +132,24 @@ struct W4Frags {
 };
 
 // LR: with a low-rank term.
-// STORE: OMX_EPI_SWIGLU and OMX_EPI_ROPE have a store pass of their own.
+// STORE: OMX_EPI_SWIGLU, OMX_EPI_ROPE and OMX_EPI_SWIGLU_BWD have a store pass of their own.
 // PAIR: B's rows are gates and, N / 2 further, ups. A wave's 128 columns are 64 units' gates and ups, which meet in its store pass: C
 // as it would be, in f32, and silu(gate) up beside it in bf16 (OMX_EPI_SWIGLU), where a pass of its own read C again. us, product and pass / so,
 // inside a step: 8192 rows over 2048 -> 2 x 8192: 490 + 112 / 545; 16384 over 768 -> 2 x 2048: 130 + 59 / 154.
 // ROPE: heads of 64 or 128 columns are turned in the store pass (OMX_EPI_ROPE), where the product went out in f32 and a pass read it: both halves of a
 // head lie in a wave's 128 columns. us, product and pass / so, inside a step: 8192 rows over
 // 2048 -> 48 heads of 128, two thirds of them turned: 213 + 51 / 204 (tables read row by row, after the staging: 241).
+// DPAIR: the product is the gradient of silu(gate) up, and gates and ups (f32, 8 N bytes a row) are read, their gradients written, in the
+// store pass (OMX_EPI_SWIGLU_BWD), where the product went out and a pass read it again. us, product and pass / so,
+// inside a step: 8192 rows over 2048 -> 8192: 225 + 147 / 359; 16384 over 768 -> 2048: 60 + 72 / 116. The 6 N bytes a row that the pass does not
+// move are what it gives; the rest moves as before, and all workgroups reach their store passes together, so beside no product.
 template <bool A_KM, bool B_KM, int TN, bool TAIL, bool LR = false, int STORE = OMX_EPI_NONE>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   static_assert(!A_KM || B_KM, "a k-major A goes with a k-major B");
   static_assert(TN == 4 || TN == 3, "256 x 256 or 256 x 192 tiles");
-  constexpr bool PAIR = STORE == OMX_EPI_SWIGLU, ROPE = STORE == OMX_EPI_ROPE;
+  constexpr bool PAIR = STORE == OMX_EPI_SWIGLU, ROPE = STORE == OMX_EPI_ROPE, DPAIR = STORE == OMX_EPI_SWIGLU_BWD;
   static_assert(!(PAIR || ROPE) || (!A_KM && !B_KM && TN == 4 && !TAIL && LR == ROPE), "one form of each");
+  static_assert(!DPAIR || (!A_KM && B_KM && TN == 4 && !TAIL && !LR), "an input gradient");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr int TM = 4, NW = 4, W4_BN = TN * 64;
   // Tile order: as gemm_dma_kernel.
@@ -462,6 +467,24 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   char* hs = reinterpret_cast<char*>(cs);
   unsigned flags = 0;  // bit 15 or 31 set: a stored bf16 has an all-ones exponent
   bool bad_act = false;
+  // DPAIR: a lane has 8 units of a row (N is a multiple of 128). Gates and ups of 16 rows are on their way while 16 others are
+  // worked on, and the barriers keep them so (each 32 rows' loads at their start, unpinned: 366 us for the 359 above).
+  float4 in[DPAIR ? 2 : 1][4][4];  // [half][row][gates, ups]
+  auto load_pairs = [&](int tm, int half) {
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const long row = min(m0 + (wm * TM + tm) * 32 + (half * 4 + it) * 4 + (lane >> 4), g.M - 1);
+      const float* gates = reinterpret_cast<const float*>(g.aux_in) + row * (2l * g.N) + gcol0 + (lane & 15) * 8;
+      in[half][it][0] = dev_stream_load<true>(reinterpret_cast<const float4*>(gates));
+      in[half][it][1] = dev_stream_load<true>(reinterpret_cast<const float4*>(gates + 4));
+      in[half][it][2] = dev_stream_load<true>(reinterpret_cast<const float4*>(gates + g.N));
+      in[half][it][3] = dev_stream_load<true>(reinterpret_cast<const float4*>(gates + g.N + 4));
+    }
+  };
+  if constexpr (DPAIR) {
+    if (gcol0 < g.N) load_pairs(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   static_for<0, TM>([&](auto tm_index) {
     constexpr int tm = decltype(tm_index)::value;
     const int grow0 = m0 + (wm * TM + tm) * 32;
@@ -547,6 +570,55 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
           }
         }
       }
+    } else if constexpr (DPAIR) {
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const floatx16& c = acc[tm][tn];
+          uint2 w;
+          w.x = dev_pack_bf16_pair(c[4 * q], c[4 * q + 1]);
+          w.y = dev_pack_bf16_pair(c[4 * q + 2], c[4 * q + 3]);
+          *reinterpret_cast<uint2*>(hs + l32 * HP + (tn * 32 + 8 * q + 4 * lg) * 2) = w;
+        }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (gcol0 < g.N) {
+        static_for<0, 2>([&](auto half_index) {
+          constexpr int half = decltype(half_index)::value;
+          if constexpr (half == 0) load_pairs(tm, 1);
+          else if constexpr (tm + 1 < TM) load_pairs(tm + 1, 0);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int it = 0; it < 4; ++it) {
+            const int row = (half * 4 + it) * 4 + (lane >> 4);
+            const uint4 v = *reinterpret_cast<const uint4*>(hs + row * HP + (lane & 15) * 16);
+            const float4* p = in[half][it];
+            const float ga[8] = {p[0].x, p[0].y, p[0].z, p[0].w, p[1].x, p[1].y, p[1].z, p[1].w};
+            const float up[8] = {p[2].x, p[2].y, p[2].z, p[2].w, p[3].x, p[3].y, p[3].z, p[3].w};
+            const unsigned w[4] = {v.x, v.y, v.z, v.w};
+            float gg[8], gu[8];
+            bool wrong = false;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float d = __uint_as_float(e & 1 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16), s = dev_sigmoid(ga[e]);
+              gu[e] = d * (ga[e] * s);
+              gg[e] = d * up[e] * (s * (1.0f + ga[e] * (1.0f - s)));
+              wrong |= !(dev_finite(gu[e]) && dev_finite(gg[e]));
+            }
+            if (grow0 + row < g.M) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) flags |= (w[e] & 0x7F807F80u) + 0x00800080u;
+              bad_act |= wrong;
+              unsigned short* to = g.aux_out + (grow0 + row) * (2l * g.N) + gcol0 + (lane & 15) * 8;
+              *reinterpret_cast<uint4*>(to) = make_uint4(dev_pack_bf16_pair(gg[0], gg[1]), dev_pack_bf16_pair(gg[2], gg[3]),
+                                                         dev_pack_bf16_pair(gg[4], gg[5]), dev_pack_bf16_pair(gg[6], gg[7]));
+              *reinterpret_cast<uint4*>(to + g.N) = make_uint4(dev_pack_bf16_pair(gu[0], gu[1]), dev_pack_bf16_pair(gu[2], gu[3]),
+                                                               dev_pack_bf16_pair(gu[4], gu[5]), dev_pack_bf16_pair(gu[6], gu[7]));
+            }
+          }
+        });
+      }
     } else if (packed && interior) {
       // bf16: rounded in registers, staged 8 bytes at a time, stored 16 bytes per lane (a wave
       // instruction writes four rows of 64 TN bytes; with TN = 3 four lanes in 16 sit out).
@@ -622,6 +694,9 @@ int32_t launch_w4(omx_ctx* ctx, const GemmArgs& g) {
   if constexpr (!A_KM && !B_KM && TN == 4) {
     if (g.epi == OMX_EPI_SWIGLU) kernel = &gemm_w4_kernel<false, false, 4, false, false, OMX_EPI_SWIGLU>;
     if (g.epi == OMX_EPI_ROPE) kernel = &gemm_w4_kernel<false, false, 4, false, true, OMX_EPI_ROPE>;
+  }
+  if constexpr (!A_KM && B_KM && TN == 4) {
+    if (g.epi == OMX_EPI_SWIGLU_BWD) kernel = &gemm_w4_kernel<false, true, 4, false, false, OMX_EPI_SWIGLU_BWD>;
   }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    W4_SMEM));

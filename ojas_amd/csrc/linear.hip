@@ -153,6 +153,21 @@ int32_t omx_linear_backward_input_gelu(omx_ctx* ctx, const void* w, const void* 
                        in_features, rows, out_features, in_features, 0, &epi);
 }
 
+// The input gradient of linear_backward followed by swiglu_backward: g_gate_up [rows, 2 hidden] (bf16) of gate_up and of gy W, w [out, hidden].
+int32_t omx_linear_backward_input_swiglu(omx_ctx* ctx, const void* w, const void* gy, int32_t operand_dtype, const void* gate_up, int32_t gate_up_dtype,
+                                         void* scratch, void* g_gate_up, uint64_t rows, uint64_t hidden, uint64_t out_features) {
+  OMX_REQUIRE_CTX(ctx);
+  const char* op = "linear_backward_input_swiglu";
+  if (!w || !gy || !gate_up || !scratch || !g_gate_up) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (operand_dtype != OMX_BF16) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: bf16 operands only", op);
+  if (rows == 0 || hidden == 0 || out_features == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
+  OmxGemmEpilogue epi = {OMX_EPI_SWIGLU_BWD, 0, gate_up, g_gate_up};
+  const bool fits = gate_up_dtype == OMX_F32;
+  const int32_t rc = omx_gemm_impl(ctx, F_LINEAR_BACKWARD, gy, out_features, 1, w, hidden, 1, OMX_BF16, scratch, OMX_BF16, hidden, rows, out_features,
+                                   hidden, 0, fits ? &epi : nullptr);
+  return rc != OMX_OK || fits ? rc : omx_swiglu_backward(ctx, gate_up, scratch, g_gate_up, gate_up_dtype, rows, hidden);
+}
+
 // The f32 tier's forms of the two: the same bits as the product and a pass over it.
 int32_t omx_linear_gelu_f32_forward(omx_ctx* ctx, const void* x, const void* w, void* u, void* act, uint64_t rows, uint64_t in_features,
                                     uint64_t out_features, int32_t tanh_form) {

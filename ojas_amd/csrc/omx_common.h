@@ -240,8 +240,10 @@ inline unsigned long long omx_tag(omx_ctx* ctx, uint32_t op) {
 //     bit as omx_swiglu_forward over C would have it; shapes without that store pass take the pass.
 //   OMX_EPI_ROPE: aux_out [m, n] (bf16) = what omx_rope_half_split_pitched makes of A.B in f32, its bits; C (f32, [m, n]) is scratch for shapes
 //     that take the pass, and is left alone otherwise.
+//   OMX_EPI_SWIGLU_BWD: aux_out [m, 2 n] (bf16) = what omx_swiglu_backward makes of aux_in [m, 2 n] (f32, gates and ups) and A.B rounded
+//     to bf16, its bits; C (bf16, [m, n]) is scratch for shapes that take the pass, and is left alone otherwise.
 // aux tensors have C's layout (pitch, and batch stride in a strided batch).
-enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3, OMX_EPI_SWIGLU = 4, OMX_EPI_ROPE = 5 };
+enum { OMX_EPI_NONE = 0, OMX_EPI_GELU_FWD = 1, OMX_EPI_GELU_BWD = 2, OMX_EPI_AXPBY = 3, OMX_EPI_SWIGLU = 4, OMX_EPI_ROPE = 5, OMX_EPI_SWIGLU_BWD = 6 };
 // The rotation of OMX_EPI_ROPE: tables [time, dim], rows are tokens of sequences of `time`, the first `heads` heads turn, `plain` follow.
 struct OmxRope {
   const float *cos_t, *sin_t;

@@ -200,8 +200,8 @@ int32_t backward(olora* t) {
   for (uint32_t l = c.layers; l-- > 0;) {
     olora::Layer& A = t->layers[l];
     // x_next = x1 + down(silu(gate) * up)
-    TRY(q8_backward(t, A.dn, t->gy16, nullptr, t->gm));
-    TRY(omx_swiglu_backward(ctx, A.gu_out, t->gm, t->ggu, OMX_F32, N, Hd));
+    TRY(omx_linear_i8_group_backward_input_swiglu(ctx, A.dn.codes, A.dn.scales, 32, OMX_I8_BLOCKED, t->gy16, OMX_BF16, A.gu_out, t->gm, t->ggu, N, A.dn.kin,
+                                                  A.dn.nout));
     TRY(q8_backward(t, A.gu, t->ggu, nullptr, t->t_a));
     // Fan-in at x1: the residual branch first, then the norm branch. The bf16 copy is this layer's
     // own: the o site's weight gradients read it after the loop.

@@ -284,9 +284,10 @@ int32_t backward(onano* t, float loss_seed) {
     // Weight gradients go to the arena now, or wait for the batched products after the loop.
     auto gw = [&](uint64_t which) { return defer ? nullptr : t->g(t->li(l, which)); };
     // x_next = x1 + down(silu(gate(h2)) * up(h2))
-    TRY(omx_linear_backward(ctx, A.m, t->w(t->li(l, FFN_DOWN)), gy, AD, t->gm, AD, gw(FFN_DOWN), OMX_F32, N, Hd, d));
+    if (defer) TRY(omx_linear_backward_input_swiglu(ctx, t->w(t->li(l, FFN_DOWN)), gy, AD, A.gu, LD, t->gm, ggu, N, Hd, d));
+    else TRY(omx_linear_backward(ctx, A.m, t->w(t->li(l, FFN_DOWN)), gy, AD, t->gm, AD, gw(FFN_DOWN), OMX_F32, N, Hd, d));
     if (t->fused_mlp) {
-      TRY(omx_swiglu_backward(ctx, A.gu, t->gm, ggu, LD, N, Hd));
+      if (!defer) TRY(omx_swiglu_backward(ctx, A.gu, t->gm, ggu, LD, N, Hd));
       // One product for both projections: their input gradients add in its f32 accumulators.
       TRY(omx_linear_backward(ctx, A.h2, t->w(t->li(l, FFN_GATE)), ggu, AD, t->t_a, AD, gw(FFN_GATE), OMX_F32, N, d,
                               2 * Hd));

@@ -469,7 +469,7 @@ struct Symbol {
   X(omx_gelu_forward) X(omx_gelu_backward) X(omx_cached_attention_forward) X(omx_kv_cache_write) X(omx_token_windows)    \
   X(omx_permute_0213) X(omx_silu_forward) X(omx_silu_backward) X(omx_mul_forward) X(omx_mul_backward) X(omx_silu_mul_forward) X(omx_silu_mul_backward)                    \
   X(omx_rope_half_split_forward) X(omx_rope_half_split_backward) X(omx_rope_half_split_inplace)                          \
-  X(omx_rope_half_split_pitched) X(omx_swiglu_forward) X(omx_swiglu_backward) X(omx_linear_swiglu_forward) X(omx_linear_i8_group_swiglu_forward) X(omx_linear_i8_group_rope_forward) X(omx_rms_qk_norm_forward)                 \
+  X(omx_rope_half_split_pitched) X(omx_swiglu_forward) X(omx_swiglu_backward) X(omx_linear_swiglu_forward) X(omx_linear_i8_group_swiglu_forward) X(omx_linear_backward_input_swiglu) X(omx_linear_i8_group_backward_input_swiglu) X(omx_linear_i8_group_rope_forward) X(omx_rms_qk_norm_forward)                 \
   X(omx_rms_qk_norm_backward) X(omx_per_head_sigmoid_gate_forward) X(omx_per_head_sigmoid_gate_backward)                 \
   X(omx_per_head_sigmoid_gate_backward_deferred) X(omx_per_head_sigmoid_gate_input_grad_add)                             \
   X(omx_value_residual_blend_forward) X(omx_value_residual_blend_backward) X(omx_qkv_prepare_forward)                    \

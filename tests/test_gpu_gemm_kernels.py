@@ -796,6 +796,47 @@ def test_products_of_one_launch_are_in_the_profile(be):
     assert flops.value == 4.0 * 1024 * 256 * 128 + ns
 
 
+@pytest.mark.parametrize("rows,out,hidden,mode", [(300, 128, 128, 9), (256, 256, 384, 9), (1, 384, 128, 9), (513, 128, 640, 9), (300, 128, 72, 9),
+                                                 (300, 192, 128, 1), (70, 64, 8, 1), (8192, 256, 1024, 1), (9000, 128, 3968, 1)])
+def test_gradients_of_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be, rows, out, hidden, mode):
+    """linear_backward_input_swiglu, with the activation's gradient in the one-wave kernel's store pass (ragged rows, tiles half outside, a
+    product cut by rows) and where it takes the pass: as linear_backward and swiglu_backward leave it; over int8 codes too; then a
+    gradient that is the first value that is not finite."""
+    from ojas_amd.backend import BF16, F32, OjasError, _native
+
+    rng = np.random.default_rng(rows + hidden)
+    gy = be.upload(rng.normal(size=(rows, out)).astype(np.float32), BF16)
+    w = be.upload((0.2 * rng.normal(size=(out, hidden))).astype(np.float32), BF16)
+    wide = rng.normal(size=(rows, 2 * hidden)).astype(np.float32)
+    gu = be.upload(wide)
+    be.set_option("gemm_dma", mode)
+    try:
+        gm, want, got, scratch = (be.empty((rows, c * hidden), BF16) for c in (1, 2, 2, 1))
+        _native.omx_linear_backward(be._context, None, w, gy, BF16, gm, BF16, None, F32, rows, hidden, out)
+        for side, dtype in ((gu, F32), (be.upload(wide, BF16), BF16)):
+            _native.omx_swiglu_backward(be._context, side, gm, want, dtype, rows, hidden)
+            _native.omx_linear_backward_input_swiglu(be._context, w, gy, BF16, side, dtype, scratch, got, rows, hidden, out)
+            np.testing.assert_array_equal(be.download(got), be.download(want))
+        if hidden % 32 == 0 and out % 32 == 0:
+            codes, scales = rng.integers(-127, 128, (out, hidden)).astype(np.int8), rng.uniform(1e-3, 2e-3, (out, hidden // 32)).astype(np.float32)
+            codes, scales = be.upload(codes), be.upload(scales)
+            for widen in (0, 1):
+                be.set_option("q8_widen", widen)
+                _native.omx_linear_i8_group_backward_input(be._context, codes, scales, 32, 0, gy, BF16, None, None, gm, rows, hidden, out)
+                _native.omx_swiglu_backward(be._context, gu, gm, want, F32, rows, hidden)
+                _native.omx_linear_i8_group_backward_input_swiglu(be._context, codes, scales, 32, 0, gy, BF16, gu, scratch, got, rows, hidden, out)
+                np.testing.assert_array_equal(be.download(got), be.download(want))
+        large = be.upload(np.full((rows, 2 * hidden), 2.0**100, np.float32))
+        _native.omx_linear_backward_input_swiglu(be._context, be.upload(np.full((out, hidden), 2.0**30, np.float32), BF16),
+                                                 be.upload(np.full((rows, out), 2.0**10, np.float32), BF16), BF16, large, F32, scratch, got, rows, hidden,
+                                                 out)
+        with pytest.raises(OjasError):
+            be.sync()
+    finally:
+        be.set_option("gemm_dma", 1)
+        be.set_option("q8_widen", -1)
+
+
 @pytest.mark.parametrize("rows,kin,hidden,mode", [(300, 128, 64, 9), (256, 256, 192, 9), (1, 384, 128, 9), (513, 128, 320, 9), (300, 128, 72, 9),
                                                  (300, 192, 64, 1), (70, 64, 8, 1), (8192, 256, 1024, 1), (9000, 128, 1984, 1)])
 def test_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be, rows, kin, hidden, mode):
