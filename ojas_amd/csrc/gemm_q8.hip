@@ -394,36 +394,37 @@ __global__ void q8_pack_kernel(const signed char* __restrict__ src, const float*
   }
 }
 
-// The weight as bf16, row-major: what gemm_q8_kernel widens a tile at a time. A thread takes 16 codes, eight of them the 128
-// columns of a block's row.
+// The weight as bf16, row-major: what gemm_q8_kernel widens a tile at a time. Memory bound: 3.1 bytes a weight. A thread takes 8
+// codes, sixteen of them the 128 columns of a block's row, so that a wave's store is four whole rows of 256 bytes (16 codes a thread stored
+// every other 16 bytes at a time, behind a 64-bit division each). us inside a step, so and now: 2048 x 16384 23.7, 20.9 (5.0 TB/s); 2048 x
+// 6144 11.4, 9.5; 1152 x 4864 7.3, 6.7. Codes read past the caches: the same, and slower where a step's codes stay in them (7.5).
 __global__ void q8_widen_kernel(const signed char* __restrict__ codes, const float* __restrict__ scales,
                                 unsigned short* __restrict__ out, long nout, long kin, int packed) {
-  const long pieces = nout * (kin / 16);
-  const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= pieces) return;
+  const unsigned across = static_cast<unsigned>(kin >> (packed ? 7 : 3));  // blocks or pieces of a row
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;  // (a weight has less than 2^31 codes)
+  if (i >= static_cast<unsigned>(nout * (kin / 8))) return;
   long row, p;
   if (packed) {
-    const long block = i >> 6, across = kin >> 7;
-    row = block / across * 8 + ((i >> 3) & 7);
-    p = block % across * 8 + (i & 7);
+    // A wave is half of a block's rows: one division for all of it.
+    const unsigned block = __builtin_amdgcn_readfirstlane(i >> 7), down = block / across;
+    row = down * 8 + ((i >> 4) & 7);
+    p = (block - down * across) * 16 + (i & 15);
   } else {
-    row = i / (kin / 16);
-    p = i % (kin / 16);
+    row = i / across;
+    p = i - static_cast<unsigned>(row) * across;
   }
-  const long group = p >> 1;
-  const uint4 v = *reinterpret_cast<const uint4*>(codes + (packed ? q8_packed_code_offset(row, group, kin) + (p & 1) * 16 : row * kin + p * 16));
+  const long group = p >> 2;
+  const uint2 v = *reinterpret_cast<const uint2*>(codes + (packed ? q8_packed_code_offset(row, group, kin) + (p & 3) * 8 : row * kin + p * 8));
   const float s = scales[packed ? q8_packed_scale_index(row, group, kin) : row * (kin / 32) + group];
-  const unsigned w[4] = {v.x, v.y, v.z, v.w};
-  unsigned r[8];
+  const unsigned w[2] = {v.x, v.y};
+  unsigned r[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int h = 0; h < 2; ++h)
       r[2 * j + h] = q8_pack2(static_cast<float>(static_cast<signed char>(w[j] >> (16 * h))) * s,
                               static_cast<float>(static_cast<signed char>(w[j] >> (16 * h + 8))) * s);
-  uint4* to = reinterpret_cast<uint4*>(out + row * kin + p * 16);
-  to[0] = make_uint4(r[0], r[1], r[2], r[3]);
-  to[1] = make_uint4(r[4], r[5], r[6], r[7]);
+  *reinterpret_cast<uint4*>(out + row * kin + p * 8) = make_uint4(r[0], r[1], r[2], r[3]);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -520,7 +521,7 @@ int32_t widened_product(omx_ctx* ctx, uint32_t fault_op, const Q8Args& g, uint64
   if (g.add || nout * kin * 2 > kMost || !widen_pays(ctx, rows, k, n) || !omx_gemm_takes_low_rank(ctx, g.a, k, nullptr, kin, k)) return OMX_OK;
   unsigned short* w = static_cast<unsigned short*>(omx_workspace_if_room(ctx, nout * kin * 2, kExtraSlot));
   if (!w) return OMX_OK;
-  const long pieces = static_cast<long>(nout) * static_cast<long>(kin / 16);
+  const long pieces = static_cast<long>(nout) * static_cast<long>(kin / 8);
   omx_launch(ctx, q8_widen_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, g.codes, g.scales, w,
              static_cast<long>(nout), static_cast<long>(kin), g.packed);
   OMX_LAUNCH_CHECK(ctx, "q8_widen_kernel");
