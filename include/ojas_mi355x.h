@@ -662,6 +662,16 @@ int32_t omx_per_head_sigmoid_gate_backward_deferred(
     const void* attn, int32_t attn_dtype, const void* gy, int32_t gy_dtype, const void* gates_f32,
     void* g_input, int32_t g_input_dtype, void* gz, void* g_bias_f32, void* g_attn,
     int32_t g_attn_dtype, uint64_t rows, uint64_t d_model, uint64_t heads, uint64_t head_dim);
+/* residual_add_forward (backend.rs:1165-1173) of attn and rest, both bf16 (an attention output and what its rounding dropped), into f32 and the
+ * gate over that sum, every bit as those two calls have it (the sum aligned as attn and rest are), without the sum in memory. The backward takes an f32 gy; of g_weight_f32
+ * and gz one may be null, and g_input where gz is not. */
+int32_t omx_per_head_sigmoid_gate_sum_forward(omx_ctx* ctx, const void* input, const void* weight, int32_t operand_dtype, const void* bias_f32,
+                                              const void* attn, const void* rest, void* y, int32_t y_dtype, void* gates_f32, uint64_t rows,
+                                              uint64_t d_model, uint64_t heads, uint64_t head_dim);
+int32_t omx_per_head_sigmoid_gate_sum_backward(omx_ctx* ctx, const void* input, const void* weight, int32_t operand_dtype, const void* bias_f32,
+                                               const void* attn, const void* rest, const void* gy_f32, const void* gates_f32, void* g_input,
+                                               int32_t g_input_dtype, void* g_weight_f32, void* gz, void* g_bias_f32, void* g_attn,
+                                               int32_t g_attn_dtype, uint64_t rows, uint64_t d_model, uint64_t heads, uint64_t head_dim);
 /* out_f32[r, i] = add_in[r, i] + sum_h gz[r, h] weight[h, i]: the grad_input of
  * per_head_sigmoid_gate_backward (backend.rs:1883-1905) from the gz that the deferred form hands
  * back, added to another gradient of the same input (residual_add_forward, backend.rs:1165-1173)

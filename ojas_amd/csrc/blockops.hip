@@ -218,16 +218,34 @@ __global__ __launch_bounds__(BK_THREADS) void gate_sigmoid_kernel(float* __restr
   }
   if (bad) dev_raise_fault(fault, tag);
 }
+// What the gate multiplies: attn, or (REST) attn and what its rounding dropped, added in f32. Memory bound; as a pass of its own the sum was
+// written in f32 and read again: 16384 rows of 12 x 64, sum and pass / so, us inside a step: forward 18 + 13.4 / 13.6,
+// backward 18 + 31.6 / 38.3.
+template <typename TA, int V, bool REST>
+__device__ __forceinline__ bool load_gated(const TA* attn, const TA* rest, size_t p, float (&a)[V]) {
+  load_pack<TA, V>(attn, p, a);
+  bool bad = false;
+  if constexpr (REST) {
+    float b[V];
+    load_pack<TA, V>(rest, p, b);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      a[j] = a[j] + b[j];
+      bad |= !dev_finite(a[j]);
+    }
+  }
+  return bad;
+}
 // y[r, h, :] = attn[r, h, :] * gates[r, h]; head_dim is a multiple of V.
-template <typename TA, typename TY, int V>
-__global__ __launch_bounds__(BK_THREADS) void gate_apply_kernel(const TA* __restrict__ attn,
+template <typename TA, typename TY, int V, bool REST = false>
+__global__ __launch_bounds__(BK_THREADS) void gate_apply_kernel(const TA* __restrict__ attn, const TA* __restrict__ rest,
                                                                 const float* __restrict__ gates, TY* __restrict__ y,
                                                                 size_t packs, int head_packs, OmxFaultWord* fault,
-                                                                unsigned long long tag) {
-  bool bad = false;
+                                                                unsigned long long tag, unsigned long long sum_tag) {
+  bool bad = false, bad_sum = false;
   PACK_LOOP(p, packs) {
     float a[V], r[V];
-    load_pack<TA, V>(attn, p, a);
+    bad_sum |= load_gated<TA, V, REST>(attn, rest, p, a);
     float g = gates[quotient(p, head_packs)];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
@@ -236,6 +254,7 @@ __global__ __launch_bounds__(BK_THREADS) void gate_apply_kernel(const TA* __rest
     }
     store_pack<TY, V>(y, p, r);
   }
+  if (bad_sum) dev_raise_fault(fault, sum_tag);
   if (bad) dev_raise_fault(fault, tag);
 }
 
@@ -244,27 +263,27 @@ __global__ __launch_bounds__(BK_THREADS) void gate_apply_kernel(const TA* __rest
 // gy * attn gives gz = dot * g * (1 - g). A block covers `block_rows` whole
 // rows; once its gz values sit in LDS, thread h adds column h in row order,
 // so the bias gradient needs no atomics.
-template <typename TA, typename TG, typename TO, typename TZ, int V>
-__global__ __launch_bounds__(BK_THREADS) void gate_bwd_kernel(const TA* __restrict__ attn, const TG* __restrict__ gy,
+template <typename TA, typename TG, typename TO, typename TZ, int V, bool REST = false>
+__global__ __launch_bounds__(BK_THREADS) void gate_bwd_kernel(const TA* __restrict__ attn, const TA* __restrict__ rest, const TG* __restrict__ gy,
                                                               const float* __restrict__ gates, TO* __restrict__ g_attn,
                                                               TZ* __restrict__ gz, float* __restrict__ partial,
                                                               size_t rows, int heads, int head_packs, int group,
                                                               int block_rows, OmxFaultWord* fault,
-                                                              unsigned long long tag) {
+                                                              unsigned long long tag, unsigned long long sum_tag) {
   extern __shared__ float lds_gz[];  // [block_rows * heads]
   const int groups = BK_THREADS / group;
   const int sub = threadIdx.x / group, lane = threadIdx.x % group;
   const size_t first_row = static_cast<size_t>(blockIdx.x) * block_rows;
   const int live_rows = static_cast<int>(min(static_cast<size_t>(block_rows), rows - first_row));
   const int items = live_rows * heads;
-  bool bad = false;
+  bool bad = false, bad_sum = false;
   for (int it = sub; it < items; it += groups) {
     const size_t item = first_row * heads + it;
     const float g = gates[item];
     float dot = 0.0f;
     for (int c = lane; c < head_packs; c += group) {
       float a[V], d[V], r[V];
-      load_pack<TA, V>(attn, item * head_packs + c, a);
+      bad_sum |= load_gated<TA, V, REST>(attn, rest, item * head_packs + c, a);
       load_pack<TG, V>(gy, item * head_packs + c, d);
 #pragma unroll
       for (int j = 0; j < V; ++j) {
@@ -288,6 +307,7 @@ __global__ __launch_bounds__(BK_THREADS) void gate_bwd_kernel(const TA* __restri
     for (int r = 0; r < live_rows; ++r) s += lds_gz[r * heads + h];
     partial[static_cast<size_t>(blockIdx.x) * heads + h] = s;
   }
+  if (bad_sum) dev_raise_fault(fault, sum_tag);
   if (bad) dev_raise_fault(fault, tag);
 }
 
@@ -623,12 +643,11 @@ int32_t omx_rope_half_split_backward(omx_ctx* ctx, const void* gy, const void* c
                            heads);
 }
 
-int32_t omx_per_head_sigmoid_gate_forward(omx_ctx* ctx, const void* input, const void* weight, int32_t operand_dtype,
-                                          const void* bias, const void* attn, int32_t attn_dtype, void* y,
-                                          int32_t y_dtype, void* gates_out, uint64_t rows, uint64_t d_model,
-                                          uint64_t heads, uint64_t head_dim) {
+// `rest` (not null: attn and it are bf16): the gate multiplies their sum.
+static int32_t gate_forward_impl(omx_ctx* ctx, const char* op, const void* input, const void* weight, int32_t operand_dtype, const void* bias,
+                                 const void* attn, const void* rest, int32_t attn_dtype, void* y, int32_t y_dtype, void* gates_out,
+                                 uint64_t rows, uint64_t d_model, uint64_t heads, uint64_t head_dim) {
   OMX_REQUIRE_CTX(ctx);
-  const char* op = "per_head_sigmoid_gate_forward";
   if (!input || !weight || !bias || !attn || !y) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
   int32_t rc = check_gate(ctx, op, operand_dtype, {attn_dtype, y_dtype}, rows, d_model, heads, head_dim);
   if (rc != OMX_OK) return rc;
@@ -641,19 +660,25 @@ int32_t omx_per_head_sigmoid_gate_forward(omx_ctx* ctx, const void* input, const
   }
   rc = compute_gates(ctx, F_GATE_FORWARD, input, weight, operand_dtype, bias, gates, rows, d_model, heads);
   if (rc != OMX_OK) return rc;
-  const bool vec = head_dim % 4 == 0 && packs_of_four(4, omx_dtype_size(attn_dtype), {attn}) &&
+  const bool vec = head_dim % 4 == 0 && packs_of_four(4, omx_dtype_size(attn_dtype), {attn, rest}) &&
                    packs_of_four(4, omx_dtype_size(y_dtype), {y});
   const int v = vec ? 4 : 1;
   const size_t packs = rows * heads * (head_dim / v);
   const int head_packs = static_cast<int>(head_dim / v);
-  unsigned long long tag = omx_tag(ctx, F_GATE_FORWARD);
+  const unsigned long long sum_tag = rest ? omx_tag(ctx, F_RESIDUAL_ADD) : 0, tag = omx_tag(ctx, F_GATE_FORWARD);
   dim3 grid = pack_grid(packs);
-#define GATE_APPLY(TA, TY, V_)                                                                                    \
-  omx_launch(ctx, (gate_apply_kernel<TA, TY, V_>), grid, dim3(BK_THREADS), 0,                     \
-                     static_cast<const TA*>(attn), gates, static_cast<TY*>(y), packs, head_packs, ctx->fault, tag)
+#define GATE_APPLY_OF(TA, TY, V_, REST)                                                                           \
+  omx_launch(ctx, (gate_apply_kernel<TA, TY, V_, REST>), grid, dim3(BK_THREADS), 0, static_cast<const TA*>(attn), \
+                     static_cast<const TA*>(rest), gates, static_cast<TY*>(y), packs, head_packs, ctx->fault, tag, sum_tag)
+#define GATE_APPLY(TA, TY, V_) GATE_APPLY_OF(TA, TY, V_, false)
   typedef unsigned short h16;
   const int key = (attn_dtype == OMX_BF16 ? 2 : 0) | (y_dtype == OMX_BF16 ? 1 : 0);
-  if (vec) {
+  if (rest) {
+    if (vec && y_dtype == OMX_BF16) GATE_APPLY_OF(h16, h16, 4, true);
+    else if (vec) GATE_APPLY_OF(h16, float, 4, true);
+    else if (y_dtype == OMX_BF16) GATE_APPLY_OF(h16, h16, 1, true);
+    else GATE_APPLY_OF(h16, float, 1, true);
+  } else if (vec) {
     switch (key) {
       case 0: GATE_APPLY(float, float, 4); break;
       case 1: GATE_APPLY(float, h16, 4); break;
@@ -669,18 +694,34 @@ int32_t omx_per_head_sigmoid_gate_forward(omx_ctx* ctx, const void* input, const
     }
   }
 #undef GATE_APPLY
+#undef GATE_APPLY_OF
   OMX_LAUNCH_CHECK(ctx, "gate_apply_kernel");
   return OMX_OK;
 }
 
+int32_t omx_per_head_sigmoid_gate_forward(omx_ctx* ctx, const void* input, const void* weight, int32_t operand_dtype,
+                                          const void* bias, const void* attn, int32_t attn_dtype, void* y,
+                                          int32_t y_dtype, void* gates_out, uint64_t rows, uint64_t d_model,
+                                          uint64_t heads, uint64_t head_dim) {
+  return gate_forward_impl(ctx, "per_head_sigmoid_gate_forward", input, weight, operand_dtype, bias, attn, nullptr, attn_dtype, y, y_dtype, gates_out,
+                           rows, d_model, heads, head_dim);
+}
+int32_t omx_per_head_sigmoid_gate_sum_forward(omx_ctx* ctx, const void* input, const void* weight, int32_t operand_dtype, const void* bias,
+                                              const void* attn, const void* rest, void* y, int32_t y_dtype, void* gates_out, uint64_t rows,
+                                              uint64_t d_model, uint64_t heads, uint64_t head_dim) {
+  if (ctx && !rest) return omx_fail(ctx, OMX_PLACEMENT, "per_head_sigmoid_gate_sum_forward: null device pointer");
+  return gate_forward_impl(ctx, "per_head_sigmoid_gate_sum_forward", input, weight, operand_dtype, bias, attn, rest, OMX_BF16, y, y_dtype, gates_out,
+                           rows, d_model, heads, head_dim);
+}
+
 // The backward of the gate. `g_weight` may be null (the weight gradient is then left to the caller)
-// and `gz_out` may be null (gz then lives in the workspace only).
+// and `gz_out` may be null (gz then lives in the workspace only). `rest`: as in the forward, beside an f32 gy.
 static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* input, const void* weight,
                                   int32_t operand_dtype, const void* bias, const void* attn, int32_t attn_dtype,
                                   const void* gy, int32_t gy_dtype, const void* gates_saved, void* g_input,
                                   int32_t g_input_dtype, void* g_weight, void* gz_out, void* g_bias, void* g_attn,
                                   int32_t g_attn_dtype, uint64_t rows, uint64_t d_model, uint64_t heads,
-                                  uint64_t head_dim) {
+                                  uint64_t head_dim, const void* rest = nullptr) {
   OMX_REQUIRE_CTX(ctx);
   // The deferred form may leave the input gradient to the caller as well (it has gz for it).
   if (!input || !weight || !bias || !attn || !gy || (!g_input && !gz_out) || !g_bias || !g_attn || (!g_weight && !gz_out))
@@ -688,7 +729,7 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
   int32_t rc = check_gate(ctx, op, operand_dtype, {attn_dtype, gy_dtype, g_input_dtype, g_attn_dtype}, rows, d_model,
                           heads, head_dim);
   if (rc != OMX_OK) return rc;
-  if (attn_dtype != gy_dtype)
+  if (rest ? gy_dtype != OMX_F32 : attn_dtype != gy_dtype)
     return omx_fail(ctx, OMX_DTYPE, "%s: attn and grad_output must share a dtype", op);
 
   // Workspace: [gates f32][gz in the operand dtype][per-block bias partials][two-stage sum scratch].
@@ -720,28 +761,40 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
   float* partial = waiting ? waiting : reinterpret_cast<float*>(base + gates_bytes + gz_bytes);
   float* stage = reinterpret_cast<float*>(base + gates_bytes + gz_bytes + partial_bytes);
 
-  const bool vec = head_dim % 4 == 0 && packs_of_four(4, omx_dtype_size(attn_dtype), {attn, gy}) &&
+  const bool vec = head_dim % 4 == 0 && packs_of_four(4, omx_dtype_size(attn_dtype), {attn, rest}) && packs_of_four(4, omx_dtype_size(gy_dtype), {gy}) &&
                    packs_of_four(4, omx_dtype_size(g_attn_dtype), {g_attn});
   const int v = vec ? 4 : 1;
   const int head_packs = static_cast<int>(head_dim / v);
   int group = 1;
   while (group < 64 && group < head_packs) group <<= 1;
-  unsigned long long tag = omx_tag(ctx, F_GATE_BACKWARD);
+  const unsigned long long sum_tag = rest ? omx_tag(ctx, F_RESIDUAL_ADD) : 0, tag = omx_tag(ctx, F_GATE_BACKWARD);
   dim3 grid(static_cast<unsigned>(blocks));
-#define GATE_BWD(TA, TO, TZ, V_)                                                                                 \
-  omx_launch(ctx, (gate_bwd_kernel<TA, TA, TO, TZ, V_>), grid, dim3(BK_THREADS), lds_bytes,      \
-                     static_cast<const TA*>(attn), static_cast<const TA*>(gy), gates, static_cast<TO*>(g_attn),  \
-                     static_cast<TZ*>(gz), partial, static_cast<size_t>(rows), static_cast<int>(heads),          \
-                     head_packs, group, block_rows, ctx->fault, tag)
+#define GATE_BWD(TA, TG, TO, TZ, V_, REST)                                                                       \
+  omx_launch(ctx, (gate_bwd_kernel<TA, TG, TO, TZ, V_, REST>), grid, dim3(BK_THREADS), lds_bytes,                \
+                     static_cast<const TA*>(attn), static_cast<const TA*>(rest), static_cast<const TG*>(gy), gates, \
+                     static_cast<TO*>(g_attn), static_cast<TZ*>(gz), partial, static_cast<size_t>(rows),         \
+                     static_cast<int>(heads), head_packs, group, block_rows, ctx->fault, tag, sum_tag)
 #define GATE_BWD_V(TA, TO, TZ)      \
   do {                              \
-    if (vec) GATE_BWD(TA, TO, TZ, 4); \
-    else GATE_BWD(TA, TO, TZ, 1);   \
+    if (vec) GATE_BWD(TA, TA, TO, TZ, 4, false); \
+    else GATE_BWD(TA, TA, TO, TZ, 1, false);   \
+  } while (0)
+#define GATE_BWD_SUM(TO, TZ)        \
+  do {                              \
+    if (vec) GATE_BWD(h16, float, TO, TZ, 4, true); \
+    else GATE_BWD(h16, float, TO, TZ, 1, true);   \
   } while (0)
   typedef unsigned short h16;
   const int key = (attn_dtype == OMX_BF16 ? 4 : 0) | (g_attn_dtype == OMX_BF16 ? 2 : 0) |
                   (operand_dtype == OMX_BF16 ? 1 : 0);
-  switch (key) {
+  if (rest) {
+    switch (key & 3) {
+      case 0: GATE_BWD_SUM(float, float); break;
+      case 1: GATE_BWD_SUM(float, h16); break;
+      case 2: GATE_BWD_SUM(h16, float); break;
+      default: GATE_BWD_SUM(h16, h16); break;
+    }
+  } else switch (key) {
     case 0: GATE_BWD_V(float, float, float); break;
     case 1: GATE_BWD_V(float, float, h16); break;
     case 2: GATE_BWD_V(float, h16, float); break;
@@ -751,6 +804,7 @@ static int32_t gate_backward_impl(omx_ctx* ctx, const char* op, const void* inpu
     case 6: GATE_BWD_V(h16, h16, float); break;
     default: GATE_BWD_V(h16, h16, h16); break;
   }
+#undef GATE_BWD_SUM
 #undef GATE_BWD_V
 #undef GATE_BWD
   OMX_LAUNCH_CHECK(ctx, "gate_bwd_kernel");
@@ -792,6 +846,16 @@ int32_t omx_per_head_sigmoid_gate_backward_deferred(omx_ctx* ctx, const void* in
   return gate_backward_impl(ctx, "per_head_sigmoid_gate_backward_deferred", input, weight, operand_dtype, bias, attn,
                             attn_dtype, gy, gy_dtype, gates_saved, g_input, g_input_dtype, nullptr, gz_out, g_bias,
                             g_attn, g_attn_dtype, rows, d_model, heads, head_dim);
+}
+
+int32_t omx_per_head_sigmoid_gate_sum_backward(omx_ctx* ctx, const void* input, const void* weight, int32_t operand_dtype, const void* bias,
+                                               const void* attn, const void* rest, const void* gy, const void* gates_saved, void* g_input,
+                                               int32_t g_input_dtype, void* g_weight, void* gz_out, void* g_bias, void* g_attn,
+                                               int32_t g_attn_dtype, uint64_t rows, uint64_t d_model, uint64_t heads, uint64_t head_dim) {
+  const char* op = "per_head_sigmoid_gate_sum_backward";
+  if (ctx && !rest) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  return gate_backward_impl(ctx, op, input, weight, operand_dtype, bias, attn, OMX_BF16, gy, OMX_F32, gates_saved, g_input, g_input_dtype, g_weight,
+                            gz_out, g_bias, g_attn, g_attn_dtype, rows, d_model, heads, head_dim, rest);
 }
 
 int32_t omx_per_head_sigmoid_gate_input_grad_add(omx_ctx* ctx, const void* gz, const void* weight, int32_t operand_dtype,

@@ -189,7 +189,7 @@ int32_t forward(olora* t) {
 int32_t backward(olora* t) {
   omx_ctx* ctx = t->ctx;
   const olora_config& c = t->c;
-  const uint64_t N = t->N, d = c.d_model, Hd = c.hidden, B = c.batch, T = c.seq, H = c.heads, D = c.head_dim, r = c.rank;
+  const uint64_t N = t->N, d = c.d_model, B = c.batch, T = c.seq, H = c.heads, D = c.head_dim, r = c.rank;
   const float eps = c.rms_eps;
   const uint64_t chunk_rows = N < 16384 ? N : 16384;
   TRY(omx_linear_cross_entropy_mean(ctx, t->hf, t->emb16, OMX_BF16, t->targets, N, d, c.vocab, 0, 0, chunk_rows, c.vocab,

@@ -91,7 +91,6 @@ struct onano {
   void *t_q = nullptr, *t_k = nullptr;   // [N, H D], [N, KV D] AD
   void *t_a = nullptr;                   // [N, max(d, H D)] AD
   void *t_f = nullptr;                   // [N, d] LD: the o and down projections' outputs on the forward
-  float *ap32 = nullptr;                 // [N, H D] f32: the attention output and its rounding residual, summed (keep_f32)
   void *gm = nullptr, *ggu = nullptr, *g_gact = nullptr, *g_up = nullptr;  // MLP gradients AD
   void *gyy = nullptr, *gap = nullptr, *gq = nullptr, *gk = nullptr, *gv = nullptr, *g_raw_v = nullptr, *part_v0 = nullptr;
   void *g_v0 = nullptr;                  // [N, KV D] AD: what the later blocks' blends send to block 0's v
@@ -212,14 +211,11 @@ int32_t forward(onano* t) {
     }
     }
     // The row-kernel attention keeps no rounding residual: the gate then reads what was stored.
-    const bool gate_f32 = t->keep_f32 && t->flash;
-    const void* attn = A.ap;
-    if (gate_f32) {  // the gate reads the attention output at 16 bits of mantissa: what was stored plus what that dropped
-      TRY(omx_residual_add(ctx, A.ap, AD, A.apr, AD, t->ap32, OMX_F32, N * qd));
-      attn = t->ap32;
-    }
-    TRY(omx_per_head_sigmoid_gate_forward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), attn,
-                                          gate_f32 ? OMX_F32 : AD, A.y, AD, A.gates, N, d, H, D));
+    if (t->keep_f32 && t->flash)  // the gate reads the attention output at 16 bits of mantissa: what was stored plus what that dropped
+      TRY(omx_per_head_sigmoid_gate_sum_forward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap, A.apr, A.y, AD, A.gates, N, d,
+                                                H, D));
+    else
+      TRY(omx_per_head_sigmoid_gate_forward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap, AD, A.y, AD, A.gates, N, d, H, D));
     TRY(omx_linear_forward(ctx, A.y, AD, t->w(t->li(l, WO)), AD, t->t_f, LD, N, qd, d));
     TRY(omx_residual_add_rms_norm_forward(ctx, A.x, OMX_F32, t->t_f, LD, t->w32(t->li(l, NORM2)), A.x1, A.h2, AD, N, d,
                                           eps));
@@ -311,20 +307,21 @@ int32_t backward(onano* t, float loss_seed) {
     // dtype: both f32 when the forward kept the output's dropped bits.
     const bool gate_f32 = t->keep_f32 && t->flash;
     const int32_t GD = gate_f32 ? OMX_F32 : AD;
-    const void* attn = A.ap;
-    if (gate_f32) {
-      TRY(omx_residual_add(ctx, A.ap, AD, A.apr, AD, t->ap32, OMX_F32, N * qd));
-      attn = t->ap32;
-    }
     TRY(omx_linear_backward(ctx, A.y, t->w(t->li(l, WO)), gy, AD, t->gyy, GD, gw(WO), OMX_F32, N, qd, d));
-    if (defer && t->gz_all)  // the gate's weight gradient waits for the batched product below
-      TRY(omx_per_head_sigmoid_gate_backward_deferred(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), attn,
-                                                      GD, t->gyy, GD, A.gates, t->fused_qkv ? nullptr : t->gh, OMX_F32,
+    const bool gz_waits = defer && t->gz_all;  // the gate's weight gradient waits for the batched product below
+    if (gate_f32)
+      TRY(omx_per_head_sigmoid_gate_sum_backward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap, A.apr, t->gyy, A.gates,
+                                                 gz_waits && t->fused_qkv ? nullptr : t->gh, OMX_F32,
+                                                 gz_waits ? nullptr : t->g(t->li(l, GATE_W)), gz_waits ? slice(t->gz_all, l, N * H) : nullptr,
+                                                 t->g(t->li(l, GATE_B)), t->gap, AD, N, d, H, D));
+    else if (gz_waits)
+      TRY(omx_per_head_sigmoid_gate_backward_deferred(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap,
+                                                      AD, t->gyy, AD, A.gates, t->fused_qkv ? nullptr : t->gh, OMX_F32,
                                                       slice(t->gz_all, l, N * H),
                                                       t->g(t->li(l, GATE_B)), t->gap, AD, N, d, H, D));
     else
-      TRY(omx_per_head_sigmoid_gate_backward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), attn, GD,
-                                             t->gyy, GD, A.gates, t->gh, OMX_F32, t->g(t->li(l, GATE_W)),
+      TRY(omx_per_head_sigmoid_gate_backward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap, AD,
+                                             t->gyy, AD, A.gates, t->gh, OMX_F32, t->g(t->li(l, GATE_W)),
                                              t->g(t->li(l, GATE_B)), t->gap, AD, N, d, H, D));
     if (t->fused_qkv) {
       const uint64_t P3 = qd + 2 * kd;
@@ -623,7 +620,6 @@ int32_t onano_create(omx_ctx* ctx, const onano_config* config, onano** out) {
   CREATE_TRY(alloc_act(t, N * kd, &t->t_k));
   CREATE_TRY(alloc_act(t, N * (d > qd ? d : qd), &t->t_a));
   CREATE_TRY(alloc(t, N * d * t->lsz, &t->t_f));
-  if (t->keep_f32 && t->flash) CREATE_TRY(alloc_t(t, N * qd, &t->ap32));
   CREATE_TRY(alloc_act(t, N * Hd, &t->gm));
   if (t->fused_mlp) {
     if (!t->deferred_dw) CREATE_TRY(alloc_act(t, 2 * N * Hd, &t->ggu));

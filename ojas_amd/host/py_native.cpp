@@ -471,7 +471,7 @@ struct Symbol {
   X(omx_rope_half_split_forward) X(omx_rope_half_split_backward) X(omx_rope_half_split_inplace)                          \
   X(omx_rope_half_split_pitched) X(omx_swiglu_forward) X(omx_swiglu_backward) X(omx_linear_swiglu_forward) X(omx_linear_i8_group_swiglu_forward) X(omx_linear_backward_input_swiglu) X(omx_linear_i8_group_backward_input_swiglu) X(omx_linear_i8_group_rope_forward) X(omx_rms_qk_norm_forward)                 \
   X(omx_rms_qk_norm_backward) X(omx_per_head_sigmoid_gate_forward) X(omx_per_head_sigmoid_gate_backward)                 \
-  X(omx_per_head_sigmoid_gate_backward_deferred) X(omx_per_head_sigmoid_gate_input_grad_add)                             \
+  X(omx_per_head_sigmoid_gate_backward_deferred) X(omx_per_head_sigmoid_gate_sum_forward) X(omx_per_head_sigmoid_gate_sum_backward) X(omx_per_head_sigmoid_gate_input_grad_add)                             \
   X(omx_value_residual_blend_forward) X(omx_value_residual_blend_backward) X(omx_qkv_prepare_forward)                    \
   X(omx_qkv_prepare_backward) X(omx_argmax_rows) X(omx_topk_rows) X(omx_set_option)
 

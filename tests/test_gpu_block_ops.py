@@ -399,6 +399,52 @@ def test_attention_saved_residual_keeps_the_row_term_exact(be, b, t, h, hkv, win
 
 
 @pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("rows,d_model,heads,head_dim,offset", [(1, 64, 1, 4, 0), (65, 96, 3, 6, 0), (300, 256, 12, 64, 0), (300, 256, 12, 64, 1),
+                                                                (4100, 128, 2, 128, 0)])
+def test_gate_over_a_sum_has_the_bits_of_sum_and_gate(be, rows, d_model, heads, head_dim, offset, bf16):
+    """The gate over an attention output and its rounding residual, added as they are read: every result of the sum as a tensor of its own
+    and the gate over that, with whole packs and without (odd heads, a residual one element off), with the weight gradient and with gz;
+    then a sum that is the first value that is not finite, named as the addition's."""
+    from ojas_amd.backend import BF16, F32, DeviceTensor, OjasError, _native
+
+    print(f"gate sum rows={rows} d={d_model} heads={heads} dim={head_dim} offset={offset} bf16={bf16}", flush=True)
+    r, n, od = orc.SplitMix64(77 + rows + head_dim), rows * heads * head_dim, BF16 if bf16 else F32
+    x, w = be.upload(r.vec(rows * d_model, 1.0).reshape(rows, d_model), BF16), be.upload(r.vec(heads * d_model, 0.2).reshape(heads, d_model), BF16)
+    b, gy = be.upload(r.vec(heads, 0.5)), be.upload(r.vec(n, 1.0))
+    attn, rest = be.upload(r.vec(n, 1.0), BF16), be.upload(r.vec(n + 8, 1e-3), BF16)
+    behind = DeviceTensor(be, rest.ptr + 2 * offset, (n,), BF16, owns=False)
+
+    def gates(names, summed):
+        room = be.empty((n + 8,), F32)  # off its packs as the residual is: a lane's elements, and so the order of a head's sum, go by that
+        total = DeviceTensor(be, room.ptr + 4 * offset, (n,), F32, owns=False)
+        _native.omx_residual_add(be._context, attn, BF16, behind, BF16, total, F32, n)
+        y, g, gi, gw, gz, gb, ga = (be.empty(shape, dt) for shape, dt in (((n,), od), ((rows, heads), F32), ((rows, d_model), F32), ((heads, d_model), F32),
+                                                                         ((rows, heads), BF16), ((heads,), F32), ((n,), od)))
+        size = (rows, d_model, heads, head_dim)
+        if summed:
+            _native.omx_per_head_sigmoid_gate_sum_forward(be._context, x, w, BF16, b, attn, behind, y, od, g, *size)
+            _native.omx_per_head_sigmoid_gate_sum_backward(be._context, x, w, BF16, b, attn, behind, gy, g, gi if names else None, F32,
+                                                           gw if names else None, None if names else gz, gb, ga, od, *size)
+        else:
+            _native.omx_per_head_sigmoid_gate_forward(be._context, x, w, BF16, b, total, F32, y, od, g, *size)
+            if names:
+                _native.omx_per_head_sigmoid_gate_backward(be._context, x, w, BF16, b, total, F32, gy, F32, g, gi, F32, gw, gb, ga, od, *size)
+            else:
+                _native.omx_per_head_sigmoid_gate_backward_deferred(be._context, x, w, BF16, b, total, F32, gy, F32, g, None, F32, gz, gb, ga, od, *size)
+        return [be.download(t) for t in ((y, g, gi, gw, gb, ga) if names else (y, g, gz, gb, ga))]
+
+    for names in (True, False):
+        for got, want in zip(gates(names, True), gates(names, False)):
+            assert np.array_equal(got, want)
+    large = be.upload(np.full(n + 8, 3.3e38, np.float32), BF16)
+    y, g = be.empty((n,), od), be.empty((rows, heads), F32)
+    _native.omx_per_head_sigmoid_gate_sum_forward(be._context, x, w, BF16, b, large, large, y, od, g, rows, d_model, heads, head_dim)
+    with pytest.raises(OjasError) as e:
+        be.sync()
+    assert "residual_add" in str(e.value.detail)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("rows,d_model,heads,head_dim", [(64, 96, 3, 8), (300, 256, 12, 64), (1024, 768, 12, 64)])
 def test_gate_backward_without_its_weight_gradient(be, rows, d_model, heads, head_dim, bf16):
     """`per_head_sigmoid_gate_backward_deferred` gives the bits of `per_head_sigmoid_gate_backward`
