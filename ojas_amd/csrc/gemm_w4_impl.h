@@ -141,8 +141,8 @@ struct W4Frags {
 // 2048 -> 48 heads of 128, two thirds of them turned: 213 + 51 / 204 (tables read row by row, after the staging: 241).
 // DPAIR: the product is the gradient of silu(gate) up, and gates and ups (f32, 8 N bytes a row) are read, their gradients written, in the
 // store pass (OMX_EPI_SWIGLU_BWD), where the product went out and a pass read it again. us, product and pass / so,
-// inside a step: 8192 rows over 2048 -> 8192: 225 + 147 / 359; 16384 over 768 -> 2048: 60 + 72 / 116. The 6 N bytes a row that the pass does not
-// move are what it gives; the rest moves as before, and all workgroups reach their store passes together, so beside no product.
+// inside a step: 8192 rows over 2048 -> 8192: 225 + 147 / 359; 16384 over 768 -> 2048: 60 + 72 / 116. The 4 N bytes a row that no longer go
+// out and back are what it gives; the rest moves as before, and all workgroups reach their store passes together, so beside no product.
 template <bool A_KM, bool B_KM, int TN, bool TAIL, bool LR = false, int STORE = OMX_EPI_NONE>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(GemmArgs g) {
   static_assert(!A_KM || B_KM, "a k-major A goes with a k-major B");
