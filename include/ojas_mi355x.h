@@ -98,7 +98,10 @@ int32_t omx_fill_zero(omx_ctx* ctx, void* dst, uint64_t bytes);
 /* Waits for all submitted work; reports and clears a deferred fault. */
 int32_t omx_sync(omx_ctx* ctx);
 /* The context's HIP stream (hipStream_t), for callers that time with events or capture graphs. The scratch that a captured op
- * used stays (charged to the budget) until the context closes; a graph is not to be replayed after that. */
+ * used stays (charged to the budget) until the context closes; a graph is not to be replayed after that. What is freed inside a
+ * capture stays too (not charged, not counted as pooled): only later captures are given it, so what one graph leaves in memory that was
+ * allocated in its capture is to be read before an earlier graph is replayed. What a capture allocated and did not free is the
+ * caller's, to be kept for as long as the graph is replayed. */
 void* omx_stream(omx_ctx* ctx);
 
 /* ---- casts: BackendCore::{cast_bf16,to_bf16,to_f32} (backend.rs:975-1090),

@@ -170,6 +170,7 @@ void omx_close(omx_ctx* ctx) {
   for (auto& kv : ctx->allocations) (void)hipFree(kv.first);
   for (auto& parked : ctx->pool)
     for (auto& block : parked.second.blocks) (void)hipFree(block.key());
+  for (auto& kept : ctx->for_graphs) (void)hipFree(kept.second.key());
   if (ctx->fault) (void)hipFree(ctx->fault);
   if (ctx->fault_host) (void)hipHostFree(ctx->fault_host);
   if (ctx->stage) (void)hipHostFree(ctx->stage);
@@ -204,10 +205,7 @@ void omx_release_pool(omx_ctx* ctx) {
   if (ctx->pooled_bytes == 0) return;
   (void)hipStreamSynchronize(ctx->stream);
   for (auto& parked : ctx->pool)
-    for (auto& block : parked.second.blocks) {
-      ctx->freed_in_capture.erase(block.key());
-      (void)hipFree(block.key());
-    }
+    for (auto& block : parked.second.blocks) (void)hipFree(block.key());
   ctx->pool.clear();
   ctx->pooled_bytes = 0;
 }
@@ -260,7 +258,6 @@ void make_room(omx_ctx* ctx, uint64_t bytes, uint64_t since) {
     auto& blocks = ctx->pool[size].blocks;
     for (size_t i = blocks.size(); i-- > 0;) {
       if (ctx->pooled_bytes + bytes <= kMaxPool - kMaxPool / 8) return;
-      if (ctx->freed_in_capture.count(blocks[i].key())) continue;
       (void)hipFree(blocks[i].key());
       blocks.erase(blocks.begin() + static_cast<std::ptrdiff_t>(i));
       ctx->pooled_bytes -= size;
@@ -287,7 +284,12 @@ int32_t omx_alloc(omx_ctx* ctx, uint64_t bytes, void** out) {
   parked.before = parked.last;
   parked.last = ++ctx->requests;
   void* p = nullptr;
-  if (!parked.blocks.empty()) {
+  auto kept = ctx->for_graphs.find(bytes);
+  if (kept != ctx->for_graphs.end() && capturing(ctx)) {
+    p = kept->second.key();
+    ctx->allocations.insert(std::move(kept->second));
+    ctx->for_graphs.erase(kept);
+  } else if (!parked.blocks.empty()) {
     // A block of this size freed earlier: every use of it is on this context's stream, so work
     // launched from here on is ordered after whatever still reads it.
     p = parked.blocks.back().key();
@@ -337,11 +339,16 @@ int32_t omx_free(omx_ctx* ctx, void* ptr) {
   // omx_alloc to a request of the same size; reuse is safe without a wait because the next user's
   // work goes onto the same stream. The pool is not charged to the budget: the budget counts what
   // callers hold.
-  const bool in_graph = capturing(ctx);
-  if (in_graph) ctx->freed_in_capture.insert(ptr);
+  if (capturing(ctx)) ctx->freed_in_capture.insert(ptr);
+  if (ctx->freed_in_capture.count(ptr)) {
+    // The graph writes this block whenever it is replayed, and nothing tells the context when that is over: never eager memory again,
+    // and not the device's either. Captures after this one take it, so that recording a graph anew needs no more.
+    ctx->for_graphs.emplace(bytes, ctx->allocations.extract(it));
+    return OMX_OK;
+  }
   if (bytes <= kMaxBlock) {
     OmxParked& parked = ctx->pool[bytes];
-    if (ctx->pooled_bytes + bytes > kMaxPool && !in_graph) make_room(ctx, bytes, parked.before);
+    if (ctx->pooled_bytes + bytes > kMaxPool) make_room(ctx, bytes, parked.before);
     if (ctx->pooled_bytes + bytes <= kMaxPool) {
       parked.blocks.push_back(ctx->allocations.extract(it));
       ctx->pooled_bytes += bytes;
@@ -349,7 +356,6 @@ int32_t omx_free(omx_ctx* ctx, void* ptr) {
     }
   }
   ctx->allocations.erase(it);
-  ctx->freed_in_capture.erase(ptr);
   OMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   OMX_HIP(ctx, hipFree(ptr));
   return OMX_OK;

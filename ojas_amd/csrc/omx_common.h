@@ -91,7 +91,10 @@ struct omx_ctx {
   // Freed blocks kept for reuse by size (see omx_free); not charged to the budget.
   std::unordered_map<uint64_t, OmxParked> pool;
   uint64_t pooled_bytes = 0, requests = 0;
-  std::set<void*> freed_in_capture;  // blocks a captured graph may still write: they stay with the context
+  // Blocks freed while the stream was captured, which a graph may still write: they stay with the context, and while no one holds them they
+  // are in for_graphs, by size, for allocations inside captures only.
+  std::set<void*> freed_in_capture;
+  std::multimap<uint64_t, std::map<void*, uint64_t>::node_type> for_graphs;
   OmxFaultWord* fault = nullptr;  // device
   OmxFaultWord* fault_host = nullptr;  // pinned, with kReadback bytes for what a small download brings behind it
   // Pinned memory that small uploads pass through (omx_upload_staged), taken by the first; up to `staged` the stream may still read it.

@@ -49,6 +49,57 @@ class Graph:
         self.hip.hipGraphDestroy(self.graph)
 
 
+def test_what_a_capture_freed_is_for_captures_only():
+    """A graph writes its temporaries whenever it is replayed: their blocks go to no eager allocation, not into the pool and, where the
+    device refuses an allocation, not back to it. A later capture takes them, and what it keeps of them and is freed afterwards is held
+    likewise."""
+    from ojas_amd.backend import MiBackend, OjasError
+
+    be = MiBackend(0)
+    n, large = (1 << 16) + 64, (256 << 18) + 64  # the second above the largest block that is parked
+    x, z = be.upload(np.full((n,), 1.5, np.float32)), be.zeros((large,))
+    inner = []
+
+    def record(t):
+        a = be.residual_add_forward(t, t)
+        inner.append(a.ptr)
+        return be.residual_add_forward(a, t)
+
+    for t, want in ((x, 4.5), (z, 0.0)):
+        inner.clear()
+        print(f"graph with a temporary of {t.nbytes} bytes", flush=True)
+        pooled, live = be.budget()["pooled"], be.budget()["live"]
+        graph = Graph(be, lambda: record(t))
+        assert be.budget()["pooled"] == pooled and be.budget()["live"] == live + t.nbytes
+        others = [be.empty(t.shape) for _ in range(2)]
+        assert inner[0] not in [o.ptr for o in others], "the temporary's block went to an eager allocation"
+        sevens = np.full(t.shape, 7.0, np.float32)
+        for o in others:
+            load(be, o, sevens)
+        graph.launch()
+        assert all(np.array_equal(be.download(o), sevens) for o in others)
+        print("a refused allocation", flush=True)
+        del others
+        with pytest.raises(OjasError):
+            be.empty((1 << 44,))
+        assert be.budget()["pooled"] == 0
+        for _ in range(3):
+            load(be, graph.results, np.full(t.shape, np.nan, np.float32))
+            graph.launch()
+            assert np.array_equal(be.download(graph.results), np.full(t.shape, want, np.float32))
+        print("a second graph", flush=True)
+        second = Graph(be, lambda: be.residual_add_forward(t, t))  # its result is the first one's temporary
+        assert second.results.ptr == inner[0]
+        second.launch()
+        assert np.array_equal(be.download(second.results), np.full(t.shape, 2.0 * want / 3.0, np.float32))
+        second.close()
+        second.results = None
+        assert be.empty(t.shape).ptr != inner[0]
+        graph.close()
+        del graph
+    be.close()
+
+
 def load(be, tensor, values):
     be._check(be._lib.omx_upload(be._ctx, be._p(tensor), C.c_uint64(0), values.ctypes.data_as(C.c_void_p), C.c_uint64(values.nbytes)))
 
