@@ -1227,16 +1227,18 @@ __global__ __launch_bounds__(AT_THREADS, D == 128 && RW == 1 ? 2 : 1) void sdpa3
   at_dkv<D, RW, false>(a, at_place(), static_cast<int>(blockIdx.z), static_cast<int>(gridDim.z), static_cast<int>(gridDim.y), lds);
 }
 
-// Both passes in one launch (at_bwd_together says when): the key side's workgroups, a part after the other, then the dQ pass's.
+// Both passes in one launch (at_bwd_together says when): the key side's workgroups, a part after the other, then the dQ pass's. The grid has
+// planes along y as those of the two passes have, so that what their launches hold this one holds (an axis takes 2^32 threads, and 16384
+// planes of 8192 positions come to 2^24 workgroups); a plane's are below 2^23, its rows of 16 values and more staying below 2^30 (at_narrow).
 template <int D>
 __global__ __launch_bounds__(AT_THREADS, 2) void sdpa32_bwd_kernel(Sdpa32Args a, unsigned planes, unsigned row_blocks, unsigned key_blocks, unsigned parts) {
   __shared__ __align__(16) float lds[at_dkv_lds<D, 4>() > at_dq_lds<D, 4>() ? at_dkv_lds<D, 4>() : at_dq_lds<D, 4>()];
-  const unsigned each = key_blocks * planes, keys = each * parts;
-  if (blockIdx.x < keys) {
-    const unsigned part = blockIdx.x / each;
-    at_dkv<D, 4, true>(a, at_place(blockIdx.x - part * each, key_blocks, planes), static_cast<int>(part), static_cast<int>(parts), static_cast<int>(planes), lds);
+  const unsigned index = blockIdx.y * gridDim.x + blockIdx.x, each = key_blocks * planes, keys = each * parts;
+  if (index < keys) {
+    const unsigned part = index / each;
+    at_dkv<D, 4, true>(a, at_place(index - part * each, key_blocks, planes), static_cast<int>(part), static_cast<int>(parts), static_cast<int>(planes), lds);
   } else {
-    at_dq<D, 4>(a, at_place(blockIdx.x - keys, row_blocks, planes), static_cast<int>(row_blocks), lds);
+    at_dq<D, 4>(a, at_place(index - keys, row_blocks, planes), static_cast<int>(row_blocks), lds);
   }
 }
 
@@ -1376,8 +1378,8 @@ int32_t backward(omx_ctx* ctx, Sdpa32Args a, int planes) {
   // dQ pass has alone (at_bwd_together).
   if (D <= 64 && narrow && row_narrow && at_bwd_together(ctx, a, planes, D)) {
     if constexpr (D <= 64)
-      omx_launch(ctx, sdpa32_bwd_kernel<D>, dim3(static_cast<unsigned>((row_blocks + blocks * parts) * planes)), dim3(AT_THREADS), 0, a, static_cast<unsigned>(planes),
-                 static_cast<unsigned>(row_blocks), static_cast<unsigned>(blocks), static_cast<unsigned>(parts));
+      omx_launch(ctx, sdpa32_bwd_kernel<D>, dim3(static_cast<unsigned>(row_blocks + blocks * parts), planes), dim3(AT_THREADS), 0, a,
+                 static_cast<unsigned>(planes), static_cast<unsigned>(row_blocks), static_cast<unsigned>(blocks), static_cast<unsigned>(parts));
     OMX_LAUNCH_CHECK(ctx, "sdpa32_bwd_kernel");
   } else {
     const dim3 row_grid(static_cast<unsigned>(row_blocks), planes), grid(static_cast<unsigned>(blocks), planes, static_cast<unsigned>(parts));

@@ -11,6 +11,8 @@ Tolerances (written where used):
   * bf16 tier: 2e-2 per element relative to max(1, max|cpu|), inputs rounded to
     bf16 on both sides so only accumulation order and output rounding differ.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -551,6 +553,30 @@ def test_f32_attention_backward_in_one_launch_has_the_bits_of_two(be, shape, hkv
             np.testing.assert_array_equal(be.download(g), e)
     finally:
         be.set_option("attention_together", -1)
+
+
+def test_f32_attention_backward_of_more_workgroups_than_an_axis_holds(be):
+    """65535 planes of 2064 positions: each pass has 2^23 workgroups and more, both together over 2^24, which are 2^32 threads (70 GB of
+    tensors, all zeros but a gradient of ones: every weight is 1, so a value's gradient counts the queries that see it)."""
+    from ojas_amd.backend import F32, DeviceTensor, _native
+
+    planes, t, d, window = 65535, 2064, 16, 1009
+    print("f32 attention backward of 2^24 workgroups", flush=True)
+    shape = (1, planes, t, d)
+    q, k, v, out, gq, gk, gv = (be.zeros(shape) for _ in range(7))
+    gy = be.empty(shape)
+    flat = lambda x, at, n: DeviceTensor(be, x.ptr + 4 * at, (n,), F32, owns=False)
+    ones, per, total = be.upload(np.ones((1 << 24,), np.float32)), 1 << 24, planes * t * d
+    for at in range(0, total, per):
+        n = min(per, total - at)
+        be._check(be._lib.omx_copy(be._ctx, be._p(flat(gy, at, n)), be._p(ones), C.c_uint64(4 * n)))
+    lse = be.zeros((1, planes, t))
+    _native.omx_causal_sdpa_backward(be._context, q, k, v, out, lse, gy, F32, F32, F32, gq, gk, gv, F32, 1, planes, planes, t, d, window)
+    counts = np.minimum(window, t - np.arange(t)).astype(np.float32)
+    for plane in (0, 1, 32767, planes - 1):
+        at = plane * t * d
+        assert np.array_equal(be.download(flat(gv, at, t * d)), np.repeat(counts, d)), plane
+        assert not be.download(flat(gq, at, t * d)).any() and not be.download(flat(gk, at, t * d)).any(), plane
 
 
 @pytest.mark.parametrize("b,h,hkv,t,d,window,tiled", [(2, 4, 2, 70, 64, 0, 0), (1, 3, 3, 130, 16, 40, 0), (2, 2, 1, 65, 128, 0, 0),
