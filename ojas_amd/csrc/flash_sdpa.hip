@@ -55,7 +55,7 @@ struct FlashShape {
   // forward and dQ; key side: dK/dV). Chosen by the host when the pairs would leave workgroup
   // places empty (few planes) or, on the key side, need a half-empty second round.
   int q_single, kv_single;
-  int aligned;   // q, k, v, gradients of the output: all rows 16-byte aligned
+  int direct;    // dK/dV: time where all rows of q, k, v and the output's gradient are 16-byte aligned (tiles go straight into LDS), else 0
   int kv_parts;  // dK/dV: workgroups that share a key block's query tiles
   float scale;
   FlashStrides q, kv, o;  // q and grad_q; k, v and their gradients; out and grad_out
@@ -852,12 +852,13 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
   int coming_q0 = 0;
   float value[VALUES];
   u32x4 rsrc_q, rsrc_g;
-  auto aim = [&](bool more) {  // (past the last tile: zeros)
+  auto aim = [&](bool more) {  // (past the last tile, and of rows that are not 16-byte aligned, which arrive() copies: zeros, nothing is read)
     coming_q = next_q;
     coming_g = next_g;
     coming_q0 = next_qt * 64;
-    rsrc_q = Dma::describe(reinterpret_cast<unsigned long long>(next_q), pitch_q, more ? T - coming_q0 : 0);
-    rsrc_g = Dma::describe(reinterpret_cast<unsigned long long>(next_g), pitch_g, more ? T - coming_q0 : 0);
+    const int live = more ? s.direct - coming_q0 : 0;
+    rsrc_q = Dma::describe(reinterpret_cast<unsigned long long>(next_q), pitch_q, live);
+    rsrc_g = Dma::describe(reinterpret_cast<unsigned long long>(next_g), pitch_g, live);
     const long row = next_row + min(lane, T - 1 - coming_q0);  // (what a row past the end carries is masked)
 #pragma unroll
     for (int j = 0; j < VALUES; ++j) value[j] = (VALUES == 2 ? j : value_of) ? delta[row] : lse[row];
@@ -874,7 +875,7 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
   // The set that was on its way is complete for this wave, its rows' values with it.
   auto arrive = [&](int set) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (__builtin_expect(!s.aligned, 0)) {
+    if (__builtin_expect(s.direct == 0, 0)) {
       dma_q.copy(coming_q, s.q.rs, T - coming_q0, smem + set * SET, lane);
       dma_g.copy(coming_g, s.o.rs, T - coming_q0, smem + set * SET + TILE, lane);
     }
@@ -1328,7 +1329,7 @@ FlashShape make_shape(uint64_t batch, uint64_t heads, uint64_t kv_heads, uint64_
   s.rep = static_cast<int>(heads / kv_heads);
   s.q_single = s.kv_single = 0;
   s.kv_parts = 1;
-  s.aligned = 0;
+  s.direct = 0;
   s.scale = scale;
   return s;
 }
@@ -1575,8 +1576,9 @@ int32_t omx_flash_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, cons
                     (unsigned long long)dim);
   FlashShape s = make_shape(batch, heads, kv_heads, time, dim, window, scale, strides);
   if (int32_t rc = check_row_strides(ctx, s); rc != OMX_OK) return rc;
-  s.aligned = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(gy)) & 15u) == 0 &&
+  const bool aligned = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(gy)) & 15u) == 0 &&
               ((s.q.rs | s.q.hs | s.q.bs | s.kv.rs | s.kv.hs | s.kv.bs | s.o.rs | s.o.hs | s.o.bs) & 7) == 0;
+  s.direct = aligned ? s.time : 0;
   const long rows = static_cast<long>(batch * heads * time);
   void* ws = nullptr;
   int32_t rc = omx_workspace(ctx, rows * sizeof(float), &ws);

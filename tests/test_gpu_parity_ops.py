@@ -1083,27 +1083,38 @@ def test_causal_sdpa_bf16_with_a_key_block_s_tiles_shared_by_workgroups(be, shap
         be.set_option("flash_kv_parts", 0)
 
 
-@pytest.mark.parametrize("groups", [1, 2, 4])
+@pytest.mark.parametrize("groups,parts", [(1, 1), (2, 1), (4, 1), (1, 3)])
+@pytest.mark.parametrize("elements", [1, 2])
 @pytest.mark.parametrize("shape,hkv,window", [((1, 2, 97, 64), 1, None), ((1, 2, 130, 128), 2, 70), ((1, 4, 200, 64), 2, 33)])
-def test_causal_sdpa_bf16_backward_of_rows_that_are_not_16_byte_aligned(be, shape, hkv, window, groups):
-    """Tiles go straight into LDS only from 16-byte rows; others are copied there, and every bit of the gradients is the same."""
-    from ojas_amd.backend import BF16, DeviceTensor
+def test_causal_sdpa_bf16_backward_of_rows_that_are_not_16_byte_aligned(be, shape, hkv, window, elements, groups, parts):
+    """Tiles go straight into LDS only from 16-byte rows; others are copied there, and every bit of the gradients is the same. Gradients
+    that lie off 16 bytes themselves, in both types: the same values, and nothing in front of them or behind."""
+    from ojas_amd.backend import BF16, F32, DeviceTensor, _native
 
     b, h, t, d = shape
+    print(f"sdpa bf16 backward, {elements} elements off, {shape} over {hkv}, {groups} groups, {parts} parts", flush=True)
     rng = np.random.default_rng(t)
     x = [rng.normal(size=(b, n, t, d)).astype(np.float32) for n in (h, hkv, hkv, h)]
     aligned = [be.upload(a, BF16) for a in x]
-    wider = [be.upload(np.concatenate([np.zeros(2, np.float32), a.ravel()]), BF16) for a in x]
-    shifted = [DeviceTensor(be, w.ptr + 4, a.shape, BF16, owns=False) for w, a in zip(wider, x)]
+    wider = [be.upload(np.concatenate([np.zeros(elements, np.float32), a.ravel()]), BF16) for a in x]
+    shifted = [DeviceTensor(be, w.ptr + 2 * elements, a.shape, BF16, owns=False) for w, a in zip(wider, x)]
     be.set_option("flash_schedule", {1: 1, 2: 3, 4: 4}[groups])
+    be.set_option("flash_kv_parts", parts)
     try:
         out, lse = be.causal_sdpa_forward(*aligned[:3], window, out_dtype=BF16)
-        want = be.causal_sdpa_backward(*aligned[:3], out, lse, aligned[3], window, grad_dtype=BF16)
-        got = be.causal_sdpa_backward(*shifted[:3], out, lse, shifted[3], window, grad_dtype=BF16)
-        for a, e in zip(got, want):
-            np.testing.assert_array_equal(be.download_f32(a), be.download_f32(e))
+        for dtype, size in ((BF16, 2), (F32, 4)):
+            want = be.causal_sdpa_backward(*aligned[:3], out, lse, aligned[3], window, grad_dtype=dtype)
+            got = be.causal_sdpa_backward(*shifted[:3], out, lse, shifted[3], window, grad_dtype=dtype)
+            room = [be.upload(np.full((a.size + 16,), 7.0, np.float32), dtype) for a in x[:3]]
+            grads = [DeviceTensor(be, r.ptr + size * elements, a.shape, dtype, owns=False) for r, a in zip(room, x)]
+            _native.omx_causal_sdpa_backward(be._context, *shifted[:3], out, lse, shifted[3], BF16, BF16, BF16, *grads, dtype, b, h, hkv, t, d, window or 0)
+            for a, r, e in zip(got, room, want):
+                e = be.download_f32(e)
+                np.testing.assert_array_equal(be.download_f32(a), e)
+                np.testing.assert_array_equal(be.download_f32(r), np.concatenate([np.full(elements, 7.0), e.ravel(), np.full(16 - elements, 7.0)]))
     finally:
         be.set_option("flash_schedule", 0)
+        be.set_option("flash_kv_parts", 0)
 
 
 @pytest.mark.parametrize("dim", [64, 128])
