@@ -221,7 +221,9 @@ int32_t omx_causal_sdpa_forward(omx_ctx* ctx, const void* q, const void* k, cons
                                 uint64_t head_dim, uint64_t window);
 /* out / gy may be stored as f32 or bf16 independently of the operands (the forward writes either;
  * the reference's tensors here are always f32). With bf16 operands an f32 `out` is read in full:
- * the row term dO . O sees the unrounded output. */
+ * the row term dO . O sees the unrounded output. Where few workgroups would walk all queries, gk and gv are summed in parts, over scratch that the
+ * op can do without: their sums have another order where the budget or the device lacks that room (bf16 on the matrix units: all parts or
+ * one; f32: as many as fit), and in a capture before which no such call outside has taken it. */
 int32_t omx_causal_sdpa_backward(omx_ctx* ctx, const void* q, const void* k, const void* v,
                                  const void* out, const void* lse, const void* gy,
                                  int32_t operand_dtype, int32_t out_dtype, int32_t gy_dtype, void* gq,
@@ -740,7 +742,7 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * (default) and split a block's tiles over groups of waves where workgroups are few, 1 / 2 = always one block / always the
  * pair, 3 / 4 = always two / four groups (two at head_dim 128; the parity tests run all).
  * "flash_kv_parts": 0 = the workgroups that share a key block's query tiles in the bf16 attention backward are chosen by estimate
- * (default), 1 .. 64 = always that many, as far as there is room for their sums.
+ * (default), 1 .. 64 = always that many, or one where there is no room for their sums.
  * "attention_together": -1 = both passes of the f32 attention backward go out in one launch over short sequences (default), 0 = never,
  * 1 = wherever they can.
  * "gemm_f32_pair": -1 = both f32 gradients of omx_linear_backward go out in one launch where that is estimated to take less

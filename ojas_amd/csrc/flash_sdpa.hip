@@ -1492,11 +1492,11 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
   const int tiles = flash_tiles(s);
   const int q_groups = flash_groups(ctx, q_planes, s.time, tiles, s.window > 0, D);
   const FlashKeyPlan plan = flash_key_plan(ctx, s, D);
-  // Split where that takes less and there is room for the sums, in as many parts as there is room for.
+  // Split where that takes less and there is room for all parts' sums: a shape's gradients are summed in one of two orders, not in one for
+  // each number of parts that a budget might hold.
   const long kv_total = static_cast<long>(kv_planes) * s.time * D;
-  float* parts = nullptr;
-  for (s.kv_parts = plan.parts; s.kv_parts > 1; --s.kv_parts)
-    if ((parts = static_cast<float*>(omx_workspace_if_room(ctx, static_cast<uint64_t>(s.kv_parts) * kv_total * 8, kExtraSlot)))) break;
+  float* const parts = plan.parts > 1 ? static_cast<float*>(omx_workspace_if_room(ctx, static_cast<uint64_t>(plan.parts) * kv_total * 8, kExtraSlot)) : nullptr;
+  s.kv_parts = parts ? plan.parts : 1;
   const int kv_groups = s.kv_parts > 1 ? plan.groups : plan.whole_groups;
   const unsigned q_rows = 128 / q_groups, kv_rows = 128 / kv_groups;
   s.q_single = q_groups > 1 || flash_single(ctx, pairs * q_planes, D == 64 ? 3 : 2, false);

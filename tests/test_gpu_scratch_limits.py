@@ -436,3 +436,31 @@ def test_attention_backward_without_room_for_shares_of_the_key_sums():
     split = [be.download_f32(g) for g in be.causal_sdpa_backward(q, k, v, out, lse, gy, None, BF16)]
     assert not all(np.array_equal(a, e) for a, e in zip(split, whole))
     be.close()
+
+
+def test_shares_of_the_key_sums_are_all_or_none():
+    """Room for some of the shares only: the bits are those of one workgroup's walk, and not of as many shares as fit."""
+    from ojas_amd.backend import BF16, MiBackend
+
+    print("5 shares of 1.5 MiB, room for 4 MiB", flush=True)
+    be = MiBackend(0, 64 << 20)
+    rng = np.random.default_rng(6)
+    q, k, v, gy = (be.upload(rng.normal(size=(1, n, 3072, 64)).astype(np.float32), BF16) for n in (4, 1, 1, 4))
+    out, lse = be.causal_sdpa_forward(q, k, v, None, BF16)
+    be.set_option("flash_schedule", 1)
+    try:
+        be.set_option("flash_kv_parts", 1)
+        whole = [be.download_f32(g) for g in be.causal_sdpa_backward(q, k, v, out, lse, gy, None, BF16)]
+        be.set_option("flash_kv_parts", 5)
+        grads = [be.empty(t.shape, BF16) for t in (q, k, v)]
+        budget = be.budget()
+        held = be.empty(((budget["limit"] - budget["live"] - (4 << 20)) // 4,))
+        del grads
+        some = [be.download_f32(g) for g in be.causal_sdpa_backward(q, k, v, out, lse, gy, None, BF16)]
+        assert all(np.array_equal(a, e) for a, e in zip(some, whole))
+        del held
+        split = [be.download_f32(g) for g in be.causal_sdpa_backward(q, k, v, out, lse, gy, None, BF16)]
+        assert not all(np.array_equal(a, e) for a, e in zip(split, whole))
+    finally:
+        be.set_option("flash_schedule", 0)
+        be.close()
