@@ -435,13 +435,19 @@ int32_t omx_rms_backward_vec(omx_ctx* ctx, const void* x, int32_t x_dtype, const
   // weight has no partial rows, and fewer rows than compute units take one each (169 x 1152: 7.6 at 8 rows, 5.0 at 4, 4.5
   // at 1; 256 x 2048 9.3, 5.5, 5.0; 2048 x 2048 14.4, 12.4). Over many rows the time does not depend on the rows a block
   // takes between 2 and 16 per wave, and fewer blocks leave fewer partial rows to add.
-  const bool few = rows <= 768 && omx_workspace_fits(ctx, ((rows + 3) / 4 + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float));
-  int rows_per_block = !gw || few ? 4 : 8;
-  if (!gw && rows <= static_cast<uint64_t>(ctx->cu_count)) rows_per_block = 1;
-  while (rows_per_block < (dim > 1024 ? 16 : 32) && rows / rows_per_block > 512) rows_per_block *= 2;
-  const uint64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
-  // A null gw: the weight is frozen, its gradient is not formed (no partial sums, no second launch).
-  float *partial = gw ? omx_partial_rows(ctx, blocks, dim) : nullptr, *scratch = nullptr;
+  // The partial rows of few rows are halved only where a budget lacks the room for those that would be used.
+  int rows_per_block;
+  uint64_t blocks;
+  float *partial = nullptr, *scratch = nullptr;
+  for (bool few = rows <= 768;; few = false) {
+    rows_per_block = !gw || few ? 4 : 8;
+    if (!gw && rows <= static_cast<uint64_t>(ctx->cu_count)) rows_per_block = 1;
+    while (rows_per_block < (dim > 1024 ? 16 : 32) && rows / rows_per_block > 512) rows_per_block *= 2;
+    blocks = (rows + rows_per_block - 1) / rows_per_block;
+    // A null gw: the weight is frozen, its gradient is not formed (no partial sums, no second launch).
+    partial = gw ? omx_partial_rows(ctx, blocks, dim) : nullptr;
+    if (!gw || partial || !few || omx_workspace_fits(ctx, (blocks + OMX_COLUMN_SUM_GROUPS) * dim * sizeof(float))) break;
+  }
   const bool wait = partial != nullptr;
   if (gw && !wait) {
     void* ws = nullptr;

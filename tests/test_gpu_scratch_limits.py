@@ -464,3 +464,38 @@ def test_shares_of_the_key_sums_are_all_or_none():
     finally:
         be.set_option("flash_schedule", 0)
         be.close()
+
+
+@pytest.mark.parametrize("waits", [True, False])
+def test_norm_backward_of_few_rows_asks_for_the_scratch_that_it_uses(waits):
+    """768 x 1300: 192 partial rows that wait are a MiB, with the scratch of a sum that does not they are two. In a MiB the waiting sum has the
+    bits it has where nothing is scarce, and the other goes without half of its rows."""
+    from ojas_amd.backend import F32, MiBackend
+
+    print(f"norm backward 768x1300, 1 MiB, waits {waits}", flush=True)
+    r = np.random.default_rng(9)
+    x, gy = (r.standard_normal((768, 1300)).astype(np.float32) for _ in range(2))
+    w = r.normal(1, 0.1, 1300).astype(np.float32)
+    got = []
+    for mib in (0, 1):
+        be = MiBackend(0, budget_bytes=64 << 20)
+        try:
+            dx, dgy, dw, gx, gw = be.upload(x), be.upload(gy), be.upload(w), be.empty(x.shape, F32), be.zeros((1300,))
+            held = be.empty((((64 << 20) - be.budget()["live"] - (mib << 20)) // 4,)) if mib else None
+            if waits:
+                be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(1)))
+            be._check(be._lib.omx_rms_norm_backward(
+                be._ctx, be._p(dx), C.c_int32(F32), be._p(dw), be._p(dgy), C.c_int32(F32), be._p(gx), C.c_int32(F32), be._p(gw), C.c_uint64(768),
+                C.c_uint64(1300), C.c_float(1e-6)))
+            if waits:
+                be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
+            got.append((be.download(gx), be.download(gw)))
+            del held
+        finally:
+            be.close()
+    assert np.array_equal(got[0][0], got[1][0])
+    assert np.array_equal(got[0][1], got[1][1]) == waits
+    for gx, gw in got:
+        want = orc.rms_norm_backward(x, w, gy)
+        close(gx, want[0])
+        close(gw, want[1])
