@@ -801,7 +801,7 @@ def test_products_of_one_launch_are_in_the_profile(be):
 def test_gradients_of_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be, rows, out, hidden, mode):
     """linear_backward_input_swiglu, with the activation's gradient in the one-wave kernel's store pass (ragged rows, tiles half outside, a
     product cut by rows) and where it takes the pass: as linear_backward and swiglu_backward leave it; over int8 codes too; then a
-    gradient that is the first value that is not finite."""
+    gradient, and a product, that is the first value that is not finite, named as its own op's."""
     from ojas_amd.backend import BF16, F32, OjasError, _native
 
     rng = np.random.default_rng(rows + hidden)
@@ -826,12 +826,13 @@ def test_gradients_of_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be
                 _native.omx_swiglu_backward(be._context, gu, gm, want, F32, rows, hidden)
                 _native.omx_linear_i8_group_backward_input_swiglu(be._context, codes, scales, 32, 0, gy, BF16, gu, scratch, got, rows, hidden, out)
                 np.testing.assert_array_equal(be.download(got), be.download(want))
-        large = be.upload(np.full((rows, 2 * hidden), 2.0**100, np.float32))
-        _native.omx_linear_backward_input_swiglu(be._context, be.upload(np.full((out, hidden), 2.0**30, np.float32), BF16),
-                                                 be.upload(np.full((rows, out), 2.0**10, np.float32), BF16), BF16, large, F32, scratch, got, rows, hidden,
-                                                 out)
-        with pytest.raises(OjasError):
-            be.sync()
+        large, steep = be.upload(np.full((rows, 2 * hidden), 2.0**100, np.float32)), be.upload(np.full((rows, out), 2.0**10, np.float32), BF16)
+        for height, name in ((2.0**30, "mul_backward"), (2.0**120, "linear_backward")):
+            _native.omx_linear_backward_input_swiglu(be._context, be.upload(np.full((out, hidden), height, np.float32), BF16), steep, BF16, large, F32, scratch,
+                                                     got, rows, hidden, out)
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.detail == name
     finally:
         be.set_option("gemm_dma", 1)
         be.set_option("q8_widen", -1)
@@ -842,7 +843,7 @@ def test_gradients_of_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be
 def test_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be, rows, kin, hidden, mode):
     """linear_swiglu_forward, with the activation in the one-wave kernel's store pass (ragged rows, half tiles of units, a product cut by
     rows) and where it takes the pass: product and activation as linear_forward and swiglu_forward leave them; over int8 codes too; then
-    a gate whose activation is the first value that is not finite."""
+    an activation, and a product, that is the first value that is not finite, named as its own op's."""
     from ojas_amd.backend import BF16, F32, OjasError, _native
 
     rng = np.random.default_rng(rows + hidden)
@@ -871,10 +872,12 @@ def test_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be, rows, kin, 
                 np.testing.assert_array_equal(be.download(got_gu), be.download(gu))
                 np.testing.assert_array_equal(be.download(got), be.download(be.swiglu_forward(gu)))
         big = be.upload(np.full((rows, kin), 2.0**60, np.float32), BF16)
-        _native.omx_linear_swiglu_forward(be._context, big, be.upload(np.full((2 * hidden, kin), 2.0**10, np.float32), BF16), BF16, got_gu, F32, got, rows,
-                                          kin, hidden)
-        with pytest.raises(OjasError):
-            be.sync()
+        for height, name in ((2.0**10, "mul_forward"), (2.0**70, "linear_forward")):
+            _native.omx_linear_swiglu_forward(be._context, big, be.upload(np.full((2 * hidden, kin), height, np.float32), BF16), BF16, got_gu, F32, got, rows,
+                                              kin, hidden)
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.detail == name
     finally:
         be.set_option("gemm_dma", 1)
         be.set_option("q8_widen", -1)

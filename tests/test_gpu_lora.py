@@ -206,7 +206,8 @@ def test_blocked_layout_gives_the_same_products(be, rows, kin, nout):
 @pytest.mark.parametrize("ranked", [True, False])
 def test_turned_heads_of_one_product_have_the_bits_of_two_calls(be, rows, kin, time, heads, plain, dim, mode, ranked):
     """linear_i8_group_rope_forward, with the rotation in the one-wave kernel's store pass (both head widths, ragged rows, sequences that end
-    inside a row block) and where it takes the pass, over the codes and over a widened copy; then a product that is not finite."""
+    inside a row block) and where it takes the pass, over the codes and over a widened copy; then a product that is not finite and one whose
+    rotation is not, each named as its own op's."""
     from ojas_amd.backend import BF16, F32, OjasError, _native
 
     nout, rank = (heads + plain) * dim, 16
@@ -229,9 +230,19 @@ def test_turned_heads_of_one_product_have_the_bits_of_two_calls(be, rows, kin, t
                                                                          heads, plain, dim)
             call(x, scales)
             np.testing.assert_array_equal(be.download(got), be.download(want))
-        call(be.upload(np.full((rows, kin), 2.0**100, np.float32), BF16), be.upload(np.full((nout, kin // 32), 2.0**30, np.float32)))
-        with pytest.raises(OjasError):
-            be.sync()
+        def refused(a, s):
+            call(a, s)
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            return e.value.detail
+
+        assert refused(be.upload(np.full((rows, kin), 2.0**100, np.float32), BF16), be.upload(np.full((nout, kin // 32), 2.0**30, np.float32))) == "linear_forward"
+        # A head's first half 2^127, its second -2^127: with cos = sin = 1 the turned ones are 2^128 and 0.
+        half = np.where(np.arange(nout) % dim < dim // 2, 1, -1).astype(np.int8)
+        row = np.zeros((rows, kin), np.float32)
+        row[:, 0] = 2.0**60
+        codes, cos, sin = be.upload(np.repeat(half[:, None], kin, axis=1)), be.upload(np.ones((time, dim), np.float32)), be.upload(np.ones((time, dim), np.float32))
+        assert refused(be.upload(row, BF16), be.upload(np.full((nout, kin // 32), 2.0**67, np.float32))) == "rope_half_split_forward"
     finally:
         be.set_option("gemm_dma", 1)
         be.set_option("q8_widen", -1)

@@ -380,7 +380,6 @@ def test_a_full_pool_makes_room_for_a_size_that_comes_back():
     graph = Graph(be, lambda: be.residual_add_forward(be.residual_add_forward(x, x), x))
     print("4 GiB parked", flush=True)
     held = [be.empty(((200 << 18) + 1024 * k,)) for k in range(21)]
-    parked_first = held[0].ptr
     del held
     full = be.budget()["pooled"]
     assert most - (201 << 20) < full <= most
@@ -398,7 +397,11 @@ def test_a_full_pool_makes_room_for_a_size_that_comes_back():
     for _ in range(3):
         graph.launch()
         assert np.array_equal(be.download(graph.results), np.full((1 << 16,), 4.5, np.float32))
-    assert parked_first
+    print("a size that went back to the device", flush=True)
+    parked = be.budget()["pooled"]
+    old = be.empty((200 << 18,))
+    assert be.budget()["pooled"] == parked, "the pool still held the block that was asked for longest ago"
+    del old
     print("a round through more than the pool holds", flush=True)
     sizes = [(160 << 18) + 1024 * k for k in range(32)]
     hits = 0
