@@ -1,7 +1,7 @@
 // bf16 MFMA flash attention for head_dim 64 and 128: causal forward, and the backward
 // as two passes (dK/dV per key block, dQ per query block) that recompute the
 // probabilities from the saved log-sum-exp, so no T x T matrix exists and no
-// atomics are needed (the sums of one output never leave one wavefront).
+// atomics are needed (where several waves or workgroups share the tiles of one output, their sums are added in a fixed order).
 //
 // Reference semantics: ojas-cpu/src/attn.rs:176-227 (forward rows), :519-597
 // (backward from saved output and lse); the blocked CPU kernel
@@ -163,7 +163,7 @@ struct TileFetch {
     }
   }
 };
-constexpr long FLASH_MAX_ROW_STRIDE = 1L << 24;  // elements: 31 rows of it, in bytes, stay below 2^32
+constexpr long FLASH_MAX_ROW_STRIDE = 1L << 24;  // elements: 63 rows of it, in bytes, and a row's pieces stay below 2^31
 
 // The wave's index as a scalar, so that what depends on it (which tiles the wave takes, which of
 // them the diagonal cuts) is decided by scalar branches.
@@ -987,8 +987,8 @@ __global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_dkv_
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const float* __restrict__ lse, const float* __restrict__ delta, const unsigned short* __restrict__ gy,
     TO* __restrict__ gk, TO* __restrict__ gv, FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
-  // Two sets of (query tile, gradient tile, 64 log-sum-exp values, 64 row terms): the next set is
-  // stored while this one is multiplied, so a tile costs one barrier.
+  // Two sets of (query tile, gradient tile, 64 log-sum-exp values, 64 row terms): the next set comes
+  // while this one is multiplied, so a tile costs one barrier.
   __shared__ __attribute__((aligned(256))) char smem[GROUPS * 2 * flash_dkv_set(D)];
   // Early key blocks are seen by the most queries: a workgroup takes one of them and then its
   // mirror image from the back (see the forward kernel).
@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(256) void flash_parts_kernel(const float* __restric
   const long row = at / D, plane = row / s.time, b = plane / s.kv_heads;
   TO* dst = (blockIdx.y ? gv : gk) + b * s.kv.bs + (plane - b * s.kv_heads) * s.kv.hs + (row - plane * s.time) * s.kv.rs + (at - row * D);
   if constexpr (sizeof(TO) == 2) {
-    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(lo.x, lo.y), pack2(lo.z, lo.w));  // (8-byte rows, as the unsplit pass stores them)
+    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(lo.x, lo.y), pack2(lo.z, lo.w));
     *reinterpret_cast<uint2*>(dst + 4) = make_uint2(pack2(hi.x, hi.y), pack2(hi.z, hi.w));
   } else {
     *reinterpret_cast<float4*>(dst) = lo;

@@ -48,7 +48,7 @@ bool omx_gemm_dma_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain) 
 }
 
 // The one-wave-per-SIMD kernel (variants 9 and 10) also needs a k-major B with a k-major A, an even
-// number of 64-column K steps, and a store pass without an activation.
+// number of 64-column K steps, and neither GELU nor a sum in its store pass (SwiGLU, its gradient and the rotation have forms of their own there).
 bool omx_gemm_w4_eligible(const GemmArgs& g, bool a_km, bool b_km, bool plain) {
   return plain && (!a_km || b_km) && whole_steps(g, a_km, b_km, 128);
 }
