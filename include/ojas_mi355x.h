@@ -761,7 +761,8 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * vocabulary). "adamw_trust": 0 = omx_adamw_step_bounded always runs its checking pass
  * (default 1). "muon_fused_sums": 0 = the Newton-Schulz iteration forms b A + c A^2 and
  * a X + B X in kernels of their own instead of in the products' store passes (default 1; the
- * same bits either way). "sdpa_tiled": 0 = f32 attention always takes the one-wave-per-row
+ * same bits either way). "muon_symmetric": 0 = the bf16 iteration forms both halves of X X^T and b A + c A^2 (default 1: one half, stored
+ * twice, where the chip does not hold all tiles at once; the same bits). "sdpa_tiled": 0 = f32 attention always takes the one-wave-per-row
  * kernels (default 1: matrix-unit kernels at head_dim 16 / 32 / 64 / 128 with 16-byte aligned
  * f32 tensors). Results are within the same tolerances under every setting. */
 int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value);

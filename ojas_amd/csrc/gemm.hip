@@ -426,7 +426,7 @@ int dma_splits(long tiles, int ksteps) {
 // 44.2 us, of 768 x 768 over 4096: 24.7 -> 16.0); one step time for every number of tiles on a unit, and a larger tiling
 // judged at one split only, picked 6 % behind.
 double dma_us(int variant, long m, long n, long batches, int ksteps, int splits, bool a_km, bool activation, bool unaligned,
-              long cus) {
+              long cus, bool symmetric = false) {
   struct Cost {
     double base, activation, unaligned, one[2], more[2], far;  // [k-contiguous A, k-major A]
   };
@@ -437,7 +437,7 @@ double dma_us(int variant, long m, long n, long batches, int ksteps, int splits,
   const Cost& c = kCosts[variant == 3 ? 0 : variant - 5];
   int bm, bn;
   omx_gemm_dma_tile(variant, &bm, &bn);
-  const long groups = ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batches * splits;
+  const long groups = (symmetric ? omx_symmetric_tiles(m, bm, bn) : ((m + bm - 1) / bm) * ((n + bn - 1) / bn)) * batches * splits;
   const double fullest = static_cast<double>((groups + cus - 1) / cus), mean = static_cast<double>(groups) / static_cast<double>(cus);
   const double tiles = variant == 3 ? std::max(1.0, 0.5 * (fullest + mean)) : fullest;
   const double far = 1.0 + c.far * std::min(1.0, std::max(0.0, (ksteps - 32) / 224.0));
@@ -663,6 +663,10 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     if ((g.batch_a | g.batch_b | g.batch_c) & 15)
       return omx_fail(ctx, OMX_SHAPE, "%s: batch strides must be multiples of 16 bytes", op);
   }
+  // A batch of symmetric outputs: half of each is formed, on the tiling below 256 x 256 that the estimate finds cheapest.
+  const int epi_mode = epi ? epi->mode : OMX_EPI_NONE;
+  g.symmetric = batch && batch->symmetric && batches > 1 && operand_dtype == OMX_BF16 && g.c_bf16 && !accumulate && !low_rank && m == n && m >= 128 &&
+                k % 64 == 0 && a_km == b_km && (epi_mode == OMX_EPI_NONE || (epi_mode == OMX_EPI_AXPBY && !a_km));
   // Kernel choice. bf16 shapes whose output fills the chip with 256 x 256 (or
   // 256 x 128) tiles take the direct-to-LDS kernel; f32 shapes take f32_tile's choice;
   // everything else (odd shapes, small outputs that need split-K) takes the 128 x 128 kernel.
@@ -802,7 +806,26 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     else if (mode == 9) dma_variant = 9;
     else if (mode == 10) dma_variant = 10;
     if (dma_variant >= 9 && !omx_gemm_w4_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) dma_variant = 3;
+    if (g.symmetric && mode == 1 && ctx->gemm_forced_tiling < 0 && dma_variant >= 0 && dma_variant < 9) {
+      // Half the tiles of another count: which tiling fills the chip with them is asked again, and whether that is less than the whole
+      // product takes; where the chip holds all tiles at once it is not, and the second store of a tile costs 0.4 to 0.9 us. All 15
+      // products of a step, us, whole / half: 48 matrices of 768 x 768 963 / 786, 12 of 3072 x 768 621 / 550, 24 of 2048 x 768 852 /
+      // 725, 40 of 896 x 896 1219 / 948, 24 of 512 x 512 223 / 193; whole by this rule: 4 of 1024 x 256 91 / 100, 8 of 384 x 384 87 / 91.
+      auto us_of = [&](int v, bool half) {
+        return dma_us(v, g.M, g.N, g.batches, g.K / 64, 1, a_km, epi_mode != OMX_EPI_NONE, !g.c_vec, ctx->cu_count > 0 ? ctx->cu_count : 256, half);
+      };
+      int best = 3;
+      for (int v = 6; v <= 8; ++v)
+        if (us_of(v, true) < us_of(best, true)) best = v;
+      if (us_of(best, true) + 0.9 < us_of(dma_variant, false)) {
+        dma_variant = best;
+        small_splits = 1;
+      } else {
+        g.symmetric = 0;
+      }
+    }
   }
+  if (dma_variant < 0 || dma_variant >= 9 || thin || skinny) g.symmetric = 0;
   // One 256 x 256 workgroup per compute unit: when the last round of tiles fills under 2/5 of the
   // chip (the head's weight gradient: 591 tiles on 256 units), the rows of the whole rounds go to
   // this tiling and the rest to a launch of their own, which picks a smaller tile (1181 -> 1034 us).
@@ -986,6 +1009,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     OMX_HIP(ctx, take(&timed.start));
     OMX_HIP(ctx, take(&timed.stop));
     timed.flops = 2.0 * static_cast<double>(m) * static_cast<double>(n) * static_cast<double>(k) * static_cast<double>(batches);
+    if (g.symmetric) timed.flops *= static_cast<double>(omx_gemm_tiles(g, BM, BN)) / (static_cast<double>(g.tiles_m) * g.tiles_n);
     // The kernels' own dispatch timestamps: an event recorded on the stream would be one more
     // packet before and after every product (1 ms per step over 150 products).
     ctx->timing_start = timed.start;
@@ -1155,6 +1179,11 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value) {
   if (name && strcmp(name, "muon_fused_sums") == 0) {
     if (value < 0 || value > 1) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: muon_fused_sums takes 0..1");
     ctx->muon_fused_sums = static_cast<int>(value);
+    return OMX_OK;
+  }
+  if (name && strcmp(name, "muon_symmetric") == 0) {
+    if (value < 0 || value > 1) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: muon_symmetric takes 0..1");
+    ctx->muon_symmetric = static_cast<int>(value);
     return OMX_OK;
   }
   if (name && strcmp(name, "adamw_trust") == 0) {

@@ -33,7 +33,20 @@ struct GemmArgs {
   // product y - 1's. batches == 1 for a single product.
   int batches;
   long batch_a, batch_b, batch_c;
+  int symmetric;  // C (bf16, square) equals its transpose: tiles below the diagonal are not formed but stored with those above
 };
+
+// Tiles of a symmetric output of `m` rows that are formed: those not wholly below the diagonal.
+inline long omx_symmetric_tiles(long m, int bm, int bn) {
+  long kept = 0;
+  const long tiles_n = (m + bn - 1) / bn;
+  for (long i = 0; i * bm < m; ++i) kept += tiles_n - i * bm / bn;
+  return kept;
+}
+// Workgroups of a product of a batch.
+inline long omx_gemm_tiles(const GemmArgs& g, int bm, int bn) {
+  return g.symmetric ? omx_symmetric_tiles(g.M, bm, bn) : static_cast<long>(g.tiles_m) * g.tiles_n;
+}
 
 // The arguments of product `product` of a strided batch.
 __device__ __forceinline__ void gemm_select_batch(GemmArgs& g, int product) {
@@ -273,6 +286,49 @@ __device__ __forceinline__ bool gemm_epilogue_block(const GemmArgs& g, const flo
     }
   }
   return (flags & 0x80008000u) != 0;
+}
+
+// The transpose of a 32-row block of a symmetric output, COLS columns wide (bf16; plain or OMX_EPI_AXPBY, whose aux_in is
+// symmetric too): row gcol0 + i takes the staged column i, 64 contiguous bytes. The bits of the block itself, whose
+// non-finite values its own store has found.
+template <int EPI, int COLS>
+__device__ __forceinline__ void gemm_store_mirrored(const GemmArgs& g, const float* staged, int pitch, int grow0, int gcol0, int lane) {
+  constexpr int ITERS = COLS * 8 / 64;
+  unsigned short* cbase = static_cast<unsigned short*>(g.c);
+  const bool interior = grow0 + 32 <= g.M && gcol0 + COLS <= g.N && g.c_vec != 0;
+  if (interior) {
+    long off[ITERS];
+    uint2 aux[ITERS];
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+      const int c = lane + it * 64, row = c >> 3, piece = c & 7;
+      off[it] = static_cast<long>(gcol0 + row) * g.ldc + grow0 + piece * 4;
+      if constexpr (EPI == OMX_EPI_AXPBY) aux[it] = *reinterpret_cast<const uint2*>(g.aux_in + off[it]);
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+      const int c = lane + it * 64, row = c >> 3, piece = c & 7;
+      float x[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = staged[(piece * 4 + e) * pitch + row];
+      if constexpr (EPI == OMX_EPI_AXPBY) {
+        x[0] = gemm_axpby(g, __uint_as_float(aux[it].x << 16), x[0]);
+        x[1] = gemm_axpby(g, __uint_as_float(aux[it].x & 0xffff0000u), x[1]);
+        x[2] = gemm_axpby(g, __uint_as_float(aux[it].y << 16), x[2]);
+        x[3] = gemm_axpby(g, __uint_as_float(aux[it].y & 0xffff0000u), x[3]);
+      }
+      *reinterpret_cast<uint2*>(cbase + off[it]) = make_uint2(dev_pack_bf16_pair(x[0], x[1]), dev_pack_bf16_pair(x[2], x[3]));
+    }
+    return;
+  }
+#pragma unroll 1
+  for (int c = lane; c < COLS * 8; c += 64) {
+    const int row = c >> 3, piece = c & 7, grow = gcol0 + row, gcol = grow0 + piece * 4;
+    if (grow >= g.M || gcol >= g.N) continue;
+    const float* x = staged + piece * 4 * pitch + row;
+    if constexpr (EPI == OMX_EPI_AXPBY) gemm_store4_epi(g, 0, grow, gcol, x[0], x[pitch], x[2 * pitch], x[3 * pitch]);
+    else gemm_store4(g, 0, grow, gcol, x[0], x[pitch], x[2 * pitch], x[3 * pitch]);
+  }
 }
 
 // The plain store of a 32-row block that lies wholly inside the output, in the same straight-line

@@ -9,8 +9,11 @@ namespace {
 
 // EPI: the store pass (OMX_EPI_*). A kernel of its own per store pass keeps each one's code (a few KiB of
 // straight-line stores) and registers out of the others; EPI_LOW_RANK is the plain one behind a low-rank term. TAIL: see StepBase.
+// SYM: a batch of symmetric outputs (GemmArgs::symmetric), grid.x the tiles that are formed, 12 of 18 at 768 columns (128 x 128
+// tiles: 21 of 36). Bound by the matrix pipes as the whole product is; a mirrored block goes out from the staged one, 64
+// bytes a row, under the other workgroup's products. 48 x 768 x 768 over 768: 61 -> 43 us on average; where that pays: gemm.hip.
 constexpr int EPI_LOW_RANK = 16;
-template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI, bool TAIL = false>
+template <bool A_KM, bool B_KM, int WGM, int WGN, int TM, int TN, int DBK, int NST, int EPI, bool TAIL = false, bool SYM = false>
 __global__ __launch_bounds__(WGM* WGN * 64, dma_waves_per_simd(WGM* WGN, NST*(WGM* TM + WGN * TN) * 32 * DBK * 2)) void
 gemm_dma_kernel(GemmArgs g) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -31,7 +34,7 @@ gemm_dma_kernel(GemmArgs g) {
   // In a strided batch (grid.y = products, never split) an XCD takes a contiguous eighth of the
   // (product, tile) pairs instead of an eighth of every product's tiles, so a product's operands
   // are fetched into one or two L2s instead of all eight.
-  const int total = g.tiles_m * g.tiles_n;
+  const int total = SYM ? static_cast<int>(gridDim.x) : g.tiles_m * g.tiles_n;
   int split = 0, id = blockIdx.x, product = blockIdx.y;
   if (g.batches > 1 && g.splits == 1) {
     const int r = tile_of_eighth(blockIdx.y * total + blockIdx.x, total * g.batches);
@@ -43,14 +46,22 @@ gemm_dma_kernel(GemmArgs g) {
   } else {
     id = tile_of_eighth(id, total);
   }
-  const int band = 4;
-  const int tiles_per_band = band * g.tiles_n;
-  const int band_id = id / tiles_per_band;
-  const int first_m = band_id * band;
-  const int band_rows = min(band, g.tiles_m - first_m);
-  const int in_band = id - band_id * tiles_per_band;
-  const int tile_m = first_m + in_band % band_rows;
-  const int tile_n = in_band / band_rows;
+  int tile_m, tile_n;
+  if constexpr (SYM) {
+    // Row by row, each from its first tile that is not wholly below the diagonal.
+    tile_m = 0;
+    for (int kept; id >= (kept = g.tiles_n - tile_m * BM / BN); ++tile_m) id -= kept;
+    tile_n = tile_m * BM / BN + id;
+  } else {
+    const int band = 4;
+    const int tiles_per_band = band * g.tiles_n;
+    const int band_id = id / tiles_per_band;
+    const int first_m = band_id * band;
+    const int band_rows = min(band, g.tiles_m - first_m);
+    const int in_band = id - band_id * tiles_per_band;
+    tile_m = first_m + in_band % band_rows;
+    tile_n = in_band / band_rows;
+  }
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   gemm_select_batch(g, product);
   const unsigned short* __restrict__ A = static_cast<const unsigned short*>(g.a);
@@ -235,6 +246,10 @@ gemm_dma_kernel(GemmArgs g) {
         }
       }
     }
+    if constexpr (SYM) {
+      // A tile across the diagonal forms both halves itself.
+      if (n0 >= m0 + BM) gemm_store_mirrored<EPI, TN * 32>(g, cs, CPW, grow0, gcol0, lane);
+    }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   });
@@ -257,9 +272,18 @@ int32_t launch_dma(omx_ctx* ctx, const GemmArgs& g) {
   if constexpr (!A_KM) {
     if (g.lr_rank > 0) kernel = &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, EPI_LOW_RANK>;  // (whole steps)
   }
+  // (gemm.hip asks for it where A and B are read alike, whole steps, unsplit, plain or a two-term sum)
+  if constexpr (A_KM == B_KM) {
+    if (g.symmetric) {
+      kernel = &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_NONE, false, true>;
+      if constexpr (!A_KM) {
+        if (g.epi == OMX_EPI_AXPBY) kernel = &gemm_dma_kernel<A_KM, B_KM, WGM, WGN, TM, TN, DBK, NST, OMX_EPI_AXPBY, false, true>;
+      }
+    }
+  }
   OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    smem));
-  omx_launch_timed(ctx, kernel, dim3(g.tiles_m * g.tiles_n * g.splits, g.batches), dim3(WGM * WGN * 64), smem,
+  omx_launch_timed(ctx, kernel, dim3(static_cast<unsigned>(omx_gemm_tiles(g, BM, BN) * g.splits), g.batches), dim3(WGM * WGN * 64), smem,
                    ctx->timing_start, g.splits > 1 ? nullptr : ctx->timing_stop, g);
   OMX_LAUNCH_CHECK(ctx, "gemm_dma_kernel");
   return OMX_OK;
@@ -284,7 +308,7 @@ int32_t launch_variant(omx_ctx* ctx, const GemmArgs& g, int variant) {
   // chunk of 1024 rows through 12 layers of d = 768: 9.9 -> 8.6 us per product; a step of 3500 tokens at d = 512: 2.51 ->
   // 2.50 ms with 128 x 64 tiles that deep (2.43 against 2.45 before either). Repeated out of L2 short reductions take
   // 0.6 us longer, 4096 columns 1.5 us less.
-  const bool alone = static_cast<long>(g.tiles_m) * g.tiles_n * g.splits * g.batches <= (ctx->cu_count > 0 ? ctx->cu_count : 256);
+  const bool alone = omx_gemm_tiles(g, variant == 7 ? 128 : 64, 64) * g.splits * g.batches <= (ctx->cu_count > 0 ? ctx->cu_count : 256);
   if (variant == 7)
     return alone ? launch_dma<A_KM, B_KM, 2, 2, 2, 1, 64, 5>(ctx, g) : launch_dma<A_KM, B_KM, 2, 2, 2, 1, 64, 3>(ctx, g);
   if (variant == 8)

@@ -290,6 +290,10 @@ int32_t iterate_run(omx_ctx* ctx, const MuonTensors& t, const MuonWork& w, const
   const uint64_t es = L.total / sizeof(TX);  // elements between consecutive matrices' buffers
   const OmxGemmBatch batch{run.count, es, es, es};
   const OmxGemmBatch* bp = run.count > 1 ? &batch : nullptr;
+  // X X^T and the sum with its square equal their transposes.
+  OmxGemmBatch half = batch;
+  half.symmetric = ctx->muon_symmetric;
+  const OmxGemmBatch* hp = bp ? &half : nullptr;
   TX* am = reinterpret_cast<TX*>(ws + L.a);
   TX* a2 = reinterpret_cast<TX*>(ws + L.a2);
   // The two-term sums after the second and third product ride in those products' store passes (the same roundings in the same
@@ -302,12 +306,13 @@ int32_t iterate_run(omx_ctx* ctx, const MuonTensors& t, const MuonWork& w, const
     TX* xn = reinterpret_cast<TX*>(ws + (it & 1 ? L.x : L.xn));
     int32_t rc;
     // A = X' X'^T with X' the short-side-first reading of X.
-    if (!tall) rc = omx_gemm_impl(ctx, F_MUON, x, cols, 1, x, 1, cols, XD, am, XD, r, r, c, r, 0, nullptr, bp);
-    else rc = omx_gemm_impl(ctx, F_MUON, x, 1, cols, x, cols, 1, XD, am, XD, r, r, c, r, 0, nullptr, bp);
+    if (!tall) rc = omx_gemm_impl(ctx, F_MUON, x, cols, 1, x, 1, cols, XD, am, XD, r, r, c, r, 0, nullptr, hp);
+    else rc = omx_gemm_impl(ctx, F_MUON, x, 1, cols, x, cols, 1, XD, am, XD, r, r, c, r, 0, nullptr, hp);
     if (rc != OMX_OK) return rc;
     // B = b A + c A^2
     const OmxGemmEpilogue sum_b{OMX_EPI_AXPBY, 0, am, nullptr, s.b, s.c};
-    rc = omx_gemm_impl(ctx, F_MUON, am, r, 1, am, r, 1, XD, a2, XD, r, r, r, r, 0, fused ? &sum_b : nullptr, bp);
+    // (A is its own transpose: read along its rows it is B's operand too)
+    rc = omx_gemm_impl(ctx, F_MUON, am, r, 1, am, 1, r, XD, a2, XD, r, r, r, r, 0, fused ? &sum_b : nullptr, hp);
     if (rc != OMX_OK) return rc;
     if (!fused)
       omx_launch(ctx, (muon_combine_b_kernel<TX>), dim3(mu_grid(r * r), run.count), dim3(MU_THREADS), 0, t, w, s);

@@ -138,6 +138,7 @@ struct omx_ctx {
   int adamw_trust = 1;        // 0: omx_adamw_step_bounded always runs its checking pass
   int ce_fused = 1;           // 0: linear-CE always takes the separate statistics and gradient kernels
   int sdpa_tiled = 1;         // 0: f32 attention always takes the one-wave-per-row kernels
+  int muon_symmetric = 1;     // 0: bf16 Newton-Schulz forms both halves of X X^T and b A + c A^2
   int muon_fused_sums = 1;    // 0: Newton-Schulz forms b A + c A^2 and a X + B X in kernels of their own
   bool profile_gemm = false;
   uint32_t profile_classes = 0;  // bit per OmxKernelClass other than the products (omx_profile_kernels)
@@ -268,6 +269,7 @@ struct OmxGemmEpilogue {
 // `count` products of one shape whose operands lie `stride_*` ELEMENTS apart (16-byte multiples), one launch.
 struct OmxGemmBatch {
   uint64_t count, stride_a, stride_b, stride_c;
+  bool symmetric = false;  // every C equals its transpose, and aux_in too: kernels may form one half and store it twice
 };
 // `a_k`: columns of a k-contiguous A's rows that may be read, k of them and zeros after (0: just k).
 int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a_rs, uint64_t a_cs, const void* b,

@@ -430,3 +430,33 @@ def test_a_forced_kernel_takes_the_products_of_several_shapes_too(be, option, va
         be._check(be._lib.omx_profile_gemm(be._ctx, C.c_int32(0)))
         be.set_option(option, -1 if option == "gemm_f32" else 1)
     assert launches.value == 2 * 15
+
+
+@pytest.mark.parametrize("tiling", [1, 3, 4, 7, 8])
+@pytest.mark.parametrize("rows,cols,count", [(128, 128, 2), (192, 320, 3), (320, 192, 3), (448, 448, 2), (456, 576, 2), (64 * 11, 128, 4), (768, 1024, 2)])
+def test_half_formed_symmetric_products_carry_the_whole_ones_bits(be, rows, cols, count, tiling):
+    """X X^T and b A + c A^2 of a bf16 batch form one half and store it twice (`muon_symmetric`, the default): element (j, i) sums the
+    products of element (i, j) in the same order, so every bit is that of products formed whole, on every tiling, at its edges."""
+    from ojas_amd.backend import BF16, MuonNs5Config
+
+    print(f"muon symmetric {count} x {rows}x{cols}, tiling {tiling}", flush=True)
+    r = np.random.default_rng(rows + 5 * cols + count)
+    ps = [r.standard_normal((rows, cols)).astype(np.float32) * 0.1 for _ in range(count)]
+    gs = [r.standard_normal((rows, cols)).astype(np.float32) * 0.03 for _ in range(count)]
+    ms = [r.standard_normal((rows, cols)).astype(np.float32) * 0.01 for _ in range(count)]
+    got = {}
+    try:
+        be.set_option("gemm_dma", tiling)
+        for symmetric in (1, 0):
+            be.set_option("muon_symmetric", symmetric)
+            dp, dg, dm = [be.upload(x) for x in ps], [be.upload(x) for x in gs], [be.upload(x) for x in ms]
+            mirrors = [be.upload(np.zeros((rows, cols), np.float32), BF16) for _ in range(count)]
+            be.muon_ns5_step_batched(dp, dg, dm, MuonNs5Config(0.02, 0.95, 0.1, 1, 1), mirrors)
+            be.sync()
+            got[symmetric] = [be.download(t) for t in dp + dm + mirrors]
+    finally:
+        be.set_option("muon_symmetric", 1)
+        be.set_option("gemm_dma", 1)
+    for a, b in zip(got[1], got[0]):
+        assert np.array_equal(a, b)
+    assert any(np.any(a != p) for a, p in zip(got[1][:count], ps))
