@@ -351,6 +351,9 @@ int32_t omx_rms_norm_backward_residual(omx_ctx* ctx, const void* x, int32_t x_dt
  * for the size of the scratch (at most 64 MiB, given back to any allocation that would be refused, what waits formed); without
  * room they are formed at once. The reference's tape forms each where it stands (ojas-autograd/src/tape.rs:2565-2591). */
 int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected);
+/* After omx_defer_weight_sums and until omx_form_weight_sums: the weight and lambda gradients of omx_qkv_prepare_backward may wait with
+ * them. Its lambda is read when they are formed (freeing its block forms them first). */
+int32_t omx_defer_prepare_sums(omx_ctx* ctx);
 int32_t omx_form_weight_sums(omx_ctx* ctx, int32_t form);
 
 /* ---- BackendModule::cross_entropy_mean_forward / _backward

@@ -109,6 +109,7 @@ extern "C" {
     pub fn omx_residual_add_rms_norm_forward(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, y: *const c_void, y_dtype: i32, w_f32: *const c_void, sum_f32: *mut c_void, normed: *mut c_void, normed_dtype: i32, rows: u64, dim: u64, eps: f32) -> i32;
     pub fn omx_rms_norm_backward_residual(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, w_f32: *const c_void, gy: *const c_void, gy_dtype: i32, residual_grad_f32: *const c_void, gx_f32: *mut c_void, gx_bf16: *mut c_void, gw_f32: *mut c_void, rows: u64, dim: u64, eps: f32) -> i32;
     pub fn omx_defer_weight_sums(ctx: *mut OmxCtx, expected: u32) -> i32;
+    pub fn omx_defer_prepare_sums(ctx: *mut OmxCtx) -> i32;
     pub fn omx_form_weight_sums(ctx: *mut OmxCtx, form: i32) -> i32;
     pub fn omx_cross_entropy_mean_forward(ctx: *mut OmxCtx, logits: *const c_void, logits_dtype: i32, targets_u32: *const c_void, rows: u64, vocab: u64, has_ignore: i32, ignore_index: u32, loss_f32: *mut c_void) -> i32;
     pub fn omx_cross_entropy_mean_forward_static(ctx: *mut OmxCtx, logits: *const c_void, logits_dtype: i32, targets_u32: *const c_void, rows: u64, vocab: u64, has_ignore: i32, ignore_index: u32, loss_f32: *mut c_void) -> i32;

@@ -327,8 +327,8 @@ int32_t omx_free(omx_ctx* ctx, void* ptr) {
   const char* const from = static_cast<const char*>(ptr);
   const std::less<const char*> before;
   for (const OmxColumnSum& s : ctx->sums) {
-    const char* const at = reinterpret_cast<const char*>(s.out);
-    if (before(at, from) || !before(at, from + bytes)) continue;
+    auto inside = [&](const void* p) { return p && !before(static_cast<const char*>(p), from) && before(static_cast<const char*>(p), from + bytes); };
+    if (!inside(s.out) && !inside(s.blend)) continue;
     const int32_t rc = omx_form_sums(ctx);
     if (rc != OMX_OK) return rc;
     break;

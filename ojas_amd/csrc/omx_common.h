@@ -75,6 +75,7 @@ struct OmxColumnSum {
   float* out;
   unsigned long long tag;
   int blocks, dim;
+  const float* blend = nullptr;  // dim 1: out = s (1 - s) x the sum, s = sigmoid(*blend) (the gradient of a value blend's lambda)
 };
 
 // Freed blocks of one size, kept for the next request of it; the numbers of the last two requests (omx_ctx::requests).
@@ -112,7 +113,7 @@ struct omx_ctx {
   uint64_t workspace_bytes[5] = {0, 0, 0, 0, 0};
   bool extra_in_use = false;  // workspace kExtraSlot, by the op that runs
   // Column sums that wait (omx_defer_weight_sums), their partial rows in workspace kSumsSlot up to sums_used.
-  bool sums_wait = false;
+  bool sums_wait = false, prepare_sums_wait = false;
   uint32_t sums_expected = 0;
   uint64_t sums_used = 0;
   std::vector<OmxColumnSum> sums;
@@ -289,6 +290,8 @@ constexpr int OMX_COLUMN_SUM_WIDE_ROWS = 1024;
 // Sums wait in a list (`wait`) where omx_partial_rows has said so.
 int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t blocks, uint64_t dim, unsigned long long tag,
                        float* scratch = nullptr, hipEvent_t stop = nullptr, bool wait = false);
+// Sums of 17 to OMX_COLUMN_SUM_WIDE_ROWS rows (with `blend`: of any number) in one launch, or in the list where `wait`.
+int32_t omx_column_sums(omx_ctx* ctx, const OmxColumnSum* sums, int count, bool wait);
 // Where sums wait and there is room, memory for their partial rows; else null.
 float* omx_partial_rows(omx_ctx* ctx, uint64_t blocks, uint64_t dim);
 // Forms every sum that waits.
@@ -329,6 +332,13 @@ int32_t omx_convert(omx_ctx* ctx, const void* src, int32_t src_dtype, void* dst,
 // ---- device helpers ----
 typedef __hip_bfloat16 bf16_t;
 
+// sigmoid(u) and 1 - sigmoid(u), both without cancellation.
+__device__ __forceinline__ void dev_sigmoid_both(float u, float* s, float* rest) {
+  const float e = __expf(-fabsf(u));
+  const float inv = 1.0f / (1.0f + e);
+  *s = u >= 0.0f ? inv : e * inv;
+  *rest = u >= 0.0f ? e * inv : inv;
+}
 __device__ __forceinline__ float dev_sigmoid(float x) { return 1.0f / (1.0f + __expf(-x)); }
 __device__ __forceinline__ bool dev_finite(float x) {
   return (__float_as_uint(x) & 0x7fffffffu) < 0x7f800000u;

@@ -61,14 +61,6 @@ __device__ __forceinline__ float row_sum(float v) {
   if constexpr (LPR > 32) v = dev_meet_32(v, add);
   return v;
 }
-// sigmoid(u) and 1 - sigmoid(u), both without cancellation.
-__device__ __forceinline__ void sigmoid_both(float u, float* s, float* rest) {
-  const float e = __expf(-fabsf(u));
-  const float inv = 1.0f / (1.0f + e);
-  *s = u >= 0.0f ? inv : e * inv;
-  *rest = u >= 0.0f ? e * inv : inv;
-}
-
 // Row r of the launch is (token, slot): slot < heads is a query head, the next kv_heads are key
 // heads, the rest value heads.
 template <int D, typename LIN>
@@ -85,7 +77,7 @@ __global__ __launch_bounds__(QP_THREADS) void qkv_prepare_fwd_kernel(
   float blend_s = 0.0f, blend_rest = 1.0f;
   bool bad = false;
   if (v0) {
-    sigmoid_both(*lambda, &blend_s, &blend_rest);
+    dev_sigmoid_both(*lambda, &blend_s, &blend_rest);
     bad |= !dev_finite(blend_s);
   }
   for (long r = static_cast<long>(blockIdx.x) * ROWS + threadIdx.x / LPR; r < rows; r += static_cast<long>(gridDim.x) * ROWS) {
@@ -134,7 +126,7 @@ __global__ __launch_bounds__(QP_THREADS) void qkv_prepare_fwd_kernel(
 
 // The backward of the above. g is the gradient of the prepared q | k | v (same layout), g_lin that
 // of the projection output. The norm weights' gradients leave as per-workgroup partial sums
-// (partial_w: [blocks][2][D], q then k) and the blend's as one partial per workgroup; v0_acc
+// (partial_w: [2][blocks][D], q then k) and the blend's as one partial per workgroup; v0_acc
 // (f32 [tokens, kv_heads * D]) collects what the blends send to block 0's value, written when
 // `v0_first` and added to otherwise; `add_v` (block 0 only, no blend) is added to the value's gradient.
 template <int D, typename LIN>
@@ -154,7 +146,7 @@ __global__ __launch_bounds__(QP_THREADS) void qkv_prepare_bwd_kernel(
   float blend_s = 0.0f, blend_rest = 1.0f;
   bool bad = false;
   if (v0) {
-    sigmoid_both(*lambda, &blend_s, &blend_rest);
+    dev_sigmoid_both(*lambda, &blend_s, &blend_rest);
     bad |= !dev_finite(blend_s);
   }
   float acc_w[2][8];
@@ -241,32 +233,10 @@ __global__ __launch_bounds__(QP_THREADS) void qkv_prepare_bwd_kernel(
     const int which = i / D, c = i % D;
     float sum = 0.0f;
     for (int row = 0; row < ROWS; ++row) sum += red[which][row][c];
-    partial_w[(static_cast<long>(blockIdx.x) * 2 + which) * D + c] = sum;
+    partial_w[(static_cast<long>(which) * gridDim.x + blockIdx.x) * D + c] = sum;
   }
   if (threadIdx.x == 0) partial_lambda[blockIdx.x] = ((red_lambda[0] + red_lambda[1]) + red_lambda[2]) + red_lambda[3];
   if (bad) dev_raise_fault(fault, tag);
-}
-
-// g_lambda = s (1 - s) x the sum of the workgroups' partials, added in order by one workgroup.
-__global__ __launch_bounds__(256) void qkv_lambda_kernel(const float* __restrict__ partial, int blocks,
-                                                         const float* __restrict__ lambda, float* __restrict__ g_lambda,
-                                                         OmxFaultWord* fault, unsigned long long tag) {
-  __shared__ float red[256];
-  float acc = 0.0f;
-  for (int b = threadIdx.x; b < blocks; b += 256) acc += partial[b];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int step = 128; step >= 1; step >>= 1) {
-    if (threadIdx.x < step) red[threadIdx.x] += red[threadIdx.x + step];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    float s, rest;
-    sigmoid_both(*lambda, &s, &rest);
-    const float v = red[0] * s * rest;
-    if (!dev_finite(v)) dev_raise_fault(fault, tag);
-    *g_lambda = v;
-  }
 }
 
 int32_t check(omx_ctx* ctx, const char* op, uint64_t pitch, uint64_t tokens, uint64_t time, uint64_t heads,
@@ -354,14 +324,17 @@ int32_t omx_qkv_prepare_backward(omx_ctx* ctx, const void* qkv_lin, int32_t lin_
   // At most 1024 workgroups, so the partial sums stay short.
   unsigned blocks = grid_for(ctx, rows, rows_per_block);
   if (blocks > 1024) blocks = 1024;
-  void* ws = nullptr;
-  const uint64_t partial_w_floats = static_cast<uint64_t>(blocks) * 2 * head_dim;
-  rc = omx_workspace(ctx, (partial_w_floats + (1 + OMX_COLUMN_SUM_GROUPS) * 2 * head_dim + blocks + 64) * sizeof(float), &ws);
-  if (rc != OMX_OK) return rc;
-  float* partial_w = static_cast<float*>(ws);
-  float* summed = partial_w + partial_w_floats;  // [2][D]
-  float* stage = summed + 2 * head_dim;          // the column sum's first stage
-  float* partial_lambda = stage + OMX_COLUMN_SUM_GROUPS * 2 * head_dim;
+  // Rows that wait with a step driver's other sums come from there.
+  const uint64_t row_floats = 2 * head_dim + 1;
+  float* partial_w = ctx->prepare_sums_wait ? omx_partial_rows(ctx, blocks, row_floats) : nullptr;
+  const bool wait = partial_w != nullptr;
+  if (!wait) {
+    void* ws = nullptr;
+    rc = omx_workspace(ctx, blocks * row_floats * sizeof(float), &ws);
+    if (rc != OMX_OK) return rc;
+    partial_w = static_cast<float*>(ws);
+  }
+  float* partial_lambda = partial_w + blocks * 2 * head_dim;
   const unsigned long long tag = omx_tag(ctx, F_RMS_BACKWARD);
 #define QP_BWD(D_, LIN_)                                                                                               \
   omx_launch(ctx, (qkv_prepare_bwd_kernel<D_, LIN_>), dim3(blocks), dim3(QP_THREADS), 0,               \
@@ -380,19 +353,19 @@ int32_t omx_qkv_prepare_backward(omx_ctx* ctx, const void* qkv_lin, int32_t lin_
   }
 #undef QP_BWD
   OMX_LAUNCH_CHECK(ctx, "qkv_prepare_bwd_kernel");
-  // partial_w is [blocks][2 D]: one column sum gives both weights' gradients side by side.
-  rc = omx_column_sum(ctx, partial_w, summed, blocks, 2 * head_dim, tag, stage);
-  if (rc != OMX_OK) return rc;
-  rc = omx_copy(ctx, g_q_weight, summed, head_dim * sizeof(float));
-  if (rc != OMX_OK) return rc;
-  rc = omx_copy(ctx, g_k_weight, summed + head_dim, head_dim * sizeof(float));
-  if (rc != OMX_OK) return rc;
-  if (value0) {
-    omx_launch(ctx, qkv_lambda_kernel, dim3(1), dim3(256), 0, partial_lambda, static_cast<int>(blocks),
-                       static_cast<const float*>(lambda), static_cast<float*>(g_lambda), ctx->fault, tag);
-    OMX_LAUNCH_CHECK(ctx, "qkv_lambda_kernel");
+  // Both weights' gradients and lambda's go out in one launch, straight to where they belong, or wait for a step driver's. (A sum of
+  // both side by side, a copy for each and a launch for lambda were four launches of 4.7 to 7.3 us.)
+  const int n = static_cast<int>(blocks), dim = static_cast<int>(head_dim);
+  const OmxColumnSum sums[3] = {{partial_w, static_cast<float*>(g_q_weight), tag, n, dim},
+                                {partial_w + blocks * head_dim, static_cast<float*>(g_k_weight), tag, n, dim},
+                                {partial_lambda, static_cast<float*>(g_lambda), tag, n, 1, static_cast<const float*>(lambda)}};
+  const int count = value0 ? 3 : 2;
+  if (blocks > 16) return omx_column_sums(ctx, sums, count, wait);
+  for (int i = 0; i < 2; ++i) {
+    rc = omx_column_sum(ctx, sums[i].partial, sums[i].out, blocks, head_dim, tag);
+    if (rc != OMX_OK) return rc;
   }
-  return OMX_OK;
+  return omx_column_sums(ctx, sums + 2, count - 2, false);
 }
 
 }  // extern "C"

@@ -211,17 +211,40 @@ __global__ __launch_bounds__(1024) void column_sum_wide_kernel(const float* __re
   column_sum_wide(partial, out, blocks, dim, fault, tag);
 }
 
+// One column whose sum is a value blend's: 256 threads in order, then a tree.
+__device__ __forceinline__ void column_sum_blend(const OmxColumnSum& s, OmxFaultWord* fault) {
+  __shared__ float red[256];
+  if (threadIdx.x < 256) {
+    float acc = 0.0f;
+    for (int b = threadIdx.x; b < s.blocks; b += 256) acc += s.partial[b];
+    red[threadIdx.x] = acc;
+  }
+  __syncthreads();
+  for (int step = 128; step >= 1; step >>= 1) {
+    if (threadIdx.x < step) red[threadIdx.x] += red[threadIdx.x + step];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    float sig, rest;
+    dev_sigmoid_both(*s.blend, &sig, &rest);
+    const float v = red[0] * sig * rest;
+    if (!dev_finite(v)) dev_raise_fault(fault, s.tag);
+    *s.out = v;
+  }
+}
+
 // Many of them in one launch. One is 4 to 18 workgroups that wait for memory, 4 to 5 us whatever its size; the norms' of a
 // backward together take about as long as one (a step with nine norms over 2048 x 256: 1233 -> 1212 us; with thirteen over 3500 x 512:
 // 2373 -> 2346).
 constexpr int SUM_LIST = 64;
 struct ColumnSumList {
-  OmxColumnSum of[SUM_LIST];  // (2 KiB of kernel arguments)
+  OmxColumnSum of[SUM_LIST];  // (2.5 KiB of kernel arguments)
 };
 __global__ __launch_bounds__(1024) void column_sum_list_kernel(ColumnSumList list, OmxFaultWord* fault) {
   const OmxColumnSum& s = list.of[blockIdx.y];
   if (static_cast<int>(blockIdx.x) * 64 >= s.dim) return;
-  column_sum_wide(s.partial, s.out, s.blocks, s.dim, fault, s.tag);
+  if (s.blend) column_sum_blend(s, fault);
+  else column_sum_wide(s.partial, s.out, s.blocks, s.dim, fault, s.tag);
 }
 
 // Stage 1 of a tall column sum: block (x, g) adds rows [g * per_group, (g + 1) * per_group) of its
@@ -856,24 +879,32 @@ int32_t omx_column_sum(omx_ctx* ctx, const float* partial, float* out, uint64_t 
   return OMX_OK;
 }
 
-// In the kernel's order of rows; the partial rows' memory is free again behind it. Nothing waits any more if a launch fails.
-int32_t omx_form_sums(omx_ctx* ctx) {
-  const std::vector<OmxColumnSum> sums = std::exchange(ctx->sums, {});
-  ctx->sums_used = 0;
-  for (size_t first = 0; first < sums.size(); first += SUM_LIST) {
+int32_t omx_column_sums(omx_ctx* ctx, const OmxColumnSum* sums, int count, bool wait) {
+  if (wait) {
+    ctx->sums.insert(ctx->sums.end(), sums, sums + count);
+    return OMX_OK;
+  }
+  for (int first = 0; first < count; first += SUM_LIST) {
     ColumnSumList list{};
-    const size_t count = std::min<size_t>(SUM_LIST, sums.size() - first);
+    const int n = std::min(SUM_LIST, count - first);
     int dim = 0;
-    for (size_t i = 0; i < count; ++i) {
+    for (int i = 0; i < n; ++i) {
       list.of[i] = sums[first + i];
       dim = std::max(dim, list.of[i].dim);
     }
     OmxKernelTimer timer(ctx, OMX_K_RMS_BWD, 0.0);  // (the norms' own launches count the bytes)
-    omx_launch_timed(ctx, column_sum_list_kernel, dim3((dim + 63) / 64, static_cast<unsigned>(count)), dim3(1024), 0, timer.start(), timer.stop(),
+    omx_launch_timed(ctx, column_sum_list_kernel, dim3((dim + 63) / 64, static_cast<unsigned>(n)), dim3(1024), 0, timer.start(), timer.stop(),
                      list, ctx->fault);
     OMX_LAUNCH_CHECK(ctx, "column_sum_list_kernel");
   }
   return OMX_OK;
+}
+
+// In the kernel's order of rows; the partial rows' memory is free again behind it. Nothing waits any more if a launch fails.
+int32_t omx_form_sums(omx_ctx* ctx) {
+  const std::vector<OmxColumnSum> sums = std::exchange(ctx->sums, {});
+  ctx->sums_used = 0;
+  return omx_column_sums(ctx, sums.data(), static_cast<int>(sums.size()), false);
 }
 
 // The rows are those of the wide kernel, whose order the list keeps. Full memory is formed and used again. (Rows of more than 1 MiB
@@ -902,12 +933,19 @@ int32_t omx_defer_weight_sums(omx_ctx* ctx, uint32_t expected) {
   if (rc != OMX_OK) return rc;
   ctx->sums_expected = expected;
   ctx->sums_wait = true;
+  ctx->prepare_sums_wait = false;
+  return OMX_OK;
+}
+
+int32_t omx_defer_prepare_sums(omx_ctx* ctx) {
+  OMX_REQUIRE_CTX(ctx);
+  ctx->prepare_sums_wait = ctx->sums_wait;
   return OMX_OK;
 }
 
 int32_t omx_form_weight_sums(omx_ctx* ctx, int32_t form) {
   OMX_REQUIRE_CTX(ctx);
-  ctx->sums_wait = false;
+  ctx->sums_wait = ctx->prepare_sums_wait = false;
   if (form) return omx_form_sums(ctx);
   ctx->sums.clear();
   ctx->sums_used = 0;

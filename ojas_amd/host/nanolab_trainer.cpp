@@ -255,7 +255,8 @@ int32_t backward(onano* t, float loss_seed) {
     }
     TRY(omx_scale_grad(ctx, t->g(0), loss_seed, static_cast<uint64_t>(c.vocab) * d));
   }
-  WaitingSums sums(ctx, 3 * c.layers + 1);
+  WaitingSums sums(ctx, (t->fused_qkv ? 4 : 3) * c.layers + 1);
+  if (t->fused_qkv) TRY(omx_defer_prepare_sums(ctx));  // (their rows lie together)
   TRY(omx_rms_norm_backward(ctx, t->x_final, OMX_F32, t->w32(t->nf()), t->ghf, AD, t->gres, OMX_F32, t->g(t->nf()), N, d,
                             eps));
   const bool defer = t->deferred_dw;  // implies the bf16 tier

@@ -984,3 +984,37 @@ def test_weight_sums_over_a_large_batch_wait_too(rows, dim):
         assert not be.download(before).any()
     finally:
         be.close()
+
+
+@pytest.mark.parametrize("lin_f32", [False, True])
+@pytest.mark.parametrize("tokens,heads,kv_heads,dim", [(1, 2, 1, 64), (20, 12, 12, 64), (27, 3, 1, 128), (700, 6, 2, 64), (2048, 12, 12, 64)])
+def test_prepare_sums_that_wait_have_the_bits_of_those_formed_at_once(be, tokens, heads, kv_heads, dim, lin_f32):
+    """`omx_defer_prepare_sums`: the q and k norms' and lambda's gradients with a step driver's other sums, over 2 to 1024 partial rows;
+    without it they are formed at once also while the norms' wait."""
+    from ojas_amd.backend import BF16, F32
+
+    r = np.random.default_rng(tokens + heads)
+    pitch = (heads + 2 * kv_heads) * dim
+    lin, lin0 = (be.upload(r.normal(0, 1, (1, tokens, pitch)).astype(np.float32), F32 if lin_f32 else BF16) for _ in range(2))
+    g = be.upload(r.normal(0, 1, (1, tokens, pitch)).astype(np.float32), BF16)
+    qw, kw = (be.upload(r.normal(1, 0.1, dim).astype(np.float32)) for _ in range(2))
+    angles = r.normal(0, 1, (tokens, dim // 2)).astype(np.float32)
+    cos, sin = (be.upload(np.concatenate([f(angles)] * 2, axis=1)) for f in (np.cos, np.sin))
+    lam = be.upload(np.array([0.3], np.float32))
+    acc = be.zeros((1, tokens, kv_heads * dim))
+    run = lambda: be.qkv_prepare_backward(lin, g, qw, kw, cos, sin, heads, kv_heads, dim, lin0, lam, value0_grad=acc, value0_grad_first=True)
+    want = [be.download(t) for t in run()]
+    for waits in (True, False):
+        be._check(be._lib.omx_defer_weight_sums(be._ctx, C.c_uint32(2)))
+        if waits:
+            be._check(be._lib.omx_defer_prepare_sums(be._ctx))
+        got = [run(), run()]
+        if not waits:  # (a copy on the stream forms nothing)
+            before = be.empty((dim,), F32)
+            be._check(be._lib.omx_copy(be._ctx, be._p(before), be._p(got[0][1]), C.c_uint64(4 * dim)))
+        be._check(be._lib.omx_form_weight_sums(be._ctx, C.c_int32(1)))
+        for one in got:
+            for t, w in zip(one, want):
+                assert np.array_equal(be.download(t), w)
+        if not waits:
+            assert np.array_equal(be.download(before), want[1])
