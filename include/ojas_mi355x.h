@@ -746,7 +746,8 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * pair, 3 / 4 = always two / four groups (two at head_dim 128; the parity tests run all).
  * "flash_kv_parts": 0 = the workgroups that share a key block's query tiles in the bf16 attention backward are chosen by estimate
  * (default), 1 .. 64 = always that many, or one where there is no room for their sums.
- * "attention_together": -1 = both passes of the f32 attention backward go out in one launch over short sequences (default), 0 = never,
+ * "attention_together": -1 = both passes of the attention backward (f32, and bf16 with bf16 gradients) go out in one launch over short
+ * sequences (default), 0 = never,
  * 1 = wherever they can.
  * "gemm_f32_pair": -1 = both f32 gradients of omx_linear_backward go out in one launch where that is estimated to take less
  * (default), 0 = never, 1 .. 4 = always on one of four pairs of tiles, where the operands' alignment allows;

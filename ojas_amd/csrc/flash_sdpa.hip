@@ -41,6 +41,8 @@ constexpr int ftile(int D) { return 64 * fpitch(D); }   // a 64-row tile
 constexpr int FT = 256;                                 // threads per block (4 waves of 32 rows)
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr int flash_dkv_set(int D) { return 2 * 64 * D * 2 + 2 * 64 * 4; }  // bytes: query and gradient tile, two values a row
+constexpr int FLASH_OWN_ROWS = 1024;                    // row terms that a key side's workgroup keeps for itself
+constexpr int flash_dq_lds(int D, int groups) { return groups * 4 * ftile(D) + D * 4; }
 constexpr int flash_dkv_waves(int D, int groups) { return D == 64 && groups <= 2 ? 2 : 1; }
 // Waves per SIMD the query-side passes are compiled for: what their LDS leaves room for.
 constexpr int flash_waves(int D, int groups) { return groups == 1 ? (D == 64 ? 3 : 2) : groups == 2 && D == 64 ? 2 : 1; }
@@ -215,6 +217,26 @@ __device__ __forceinline__ void row_frags(const unsigned short* __restrict__ pla
   const unsigned short* at = plane + static_cast<long>(min(row, time - 1)) * rs + lg * 8;
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk) f[kk] = *reinterpret_cast<const u32x4*>(at + kk * 16);
+}
+// dO . O of the lane's row `row`, `g` its row of dO: each half-wave holds half of the row's values. (Without a residual the output is
+// read twice, so that neither load waits for the other's products.)
+template <int D>
+__device__ __forceinline__ float flash_row_delta(const u32x4 (&g)[D / 16], const unsigned short* __restrict__ out, const unsigned short* __restrict__ resid,
+                                                 long rs, int row, int time, int lg) {
+  u32x4 o[D / 16], r[D / 16];
+  row_frags<D>(out, rs, row, time, lg, o);
+  row_frags<D>(resid ? resid : out, rs, row, time, lg, r);
+  auto dot_rows = [&](const u32x4 (&x)[D / 16]) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) sum = dot_pairs(g[kk][w], x[kk][w], sum);
+    return sum;
+  };
+  float del = dot_rows(o);
+  if (resid) del += dot_rows(r);
+  return halves_sum(del);
 }
 // Row index (within a 32-row sub-tile) that accumulator register v of this lane holds.
 __device__ __forceinline__ int acc_row(int v, int lg) { return 8 * (v >> 2) + 4 * lg + (v & 3); }
@@ -792,13 +814,15 @@ struct DkvHalf {
 // GROUPS > 1: groups of the waves take the query tiles of 128 / GROUPS keys in turn, as in the forward.
 // SPLIT: the tiles of s.kv_parts workgroups are consecutive shares of the sequence over the heads, this one's is `part`, and its sums go
 // out as rows of gk and gv, each [part][b, KV head][time][D].
-template <int D, typename TO, int GROUPS, bool SPLIT>
+// OWN: delta is formed here, for the rows that see the block, in `own` (FLASH_OWN_ROWS values of LDS).
+template <int D, typename TO, int GROUPS, bool SPLIT, bool OWN = false>
 __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict__ q,
                                                 const unsigned short* __restrict__ k,
                                                 const unsigned short* __restrict__ v, const float* __restrict__ lse,
                                                 const float* __restrict__ delta, const unsigned short* __restrict__ gy,
                                                 TO* __restrict__ gk, TO* __restrict__ gv, const FlashShape& s, char* lds,
-                                                int kb, int b, int gidx, int part) {
+                                                int kb, int b, int gidx, int part, const unsigned short* __restrict__ out = nullptr,
+                                                const unsigned short* __restrict__ resid = nullptr, float* own = nullptr) {
   constexpr int ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;
   constexpr int KK = D / 16, MT = D / 32, TILE = 64 * D * 2, SET = flash_dkv_set(D);
   typedef TileDma<D, ROW_WAVES> Dma;
@@ -849,7 +873,7 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
   constexpr int VALUES = ROW_WAVES > 1 ? 1 : 2;
   const int value_of = wave & 1;  // 0: lse, 1: delta (other waves repeat them)
   const unsigned short *coming_q = next_q, *coming_g = next_g;
-  int coming_q0 = 0;
+  int coming_q0 = 0, coming_own = 0;
   float value[VALUES];
   u32x4 rsrc_q, rsrc_g;
   auto aim = [&](bool more) {  // (past the last tile, and of rows that are not 16-byte aligned, which arrive() copies: zeros, nothing is read)
@@ -861,7 +885,8 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     rsrc_g = Dma::describe(reinterpret_cast<unsigned long long>(next_g), pitch_g, live);
     const long row = next_row + min(lane, T - 1 - coming_q0);  // (what a row past the end carries is masked)
 #pragma unroll
-    for (int j = 0; j < VALUES; ++j) value[j] = (VALUES == 2 ? j : value_of) ? delta[row] : lse[row];
+    for (int j = 0; j < VALUES; ++j) value[j] = !OWN && (VALUES == 2 ? j : value_of) ? delta[row] : lse[row];
+    if constexpr (OWN) coming_own = min(next_r, s.rep - 1) * (T - qt_first * 64) + coming_q0 - qt_first * 64 + min(lane, T - 1 - coming_q0);
     for (int i = 0; i < GROUPS; ++i) skip();
   };
   auto load = [&](auto i, unsigned set) {
@@ -882,6 +907,8 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
 #pragma unroll
     for (int j = 0; j < VALUES; ++j) {
       const int which = VALUES == 2 ? j : value_of;
+      if constexpr (OWN)
+        if (which) value[j] = own[coming_own];
       *reinterpret_cast<float*>(smem + set * SET + 2 * TILE + which * 256 + lane * 4) = value[j] * (which ? 1.0f : LOG2E);
     }
   };
@@ -904,6 +931,19 @@ __device__ __forceinline__ bool flash_dkv_block(const unsigned short* __restrict
     dv[mt] = zero16();
   }
   const float scale_log2 = s.scale * LOG2E;
+  if constexpr (OWN) {
+    // The rows of tiles qt_first .. qt_last of every head of the group, 32 a wave at a time.
+    const int from = qt_first * 64, each = (min(T, qt_last * 64 + 64) - from + 31) / 32;
+    for (int n = wave_index(); n < s.rep * each; n += 4) {
+      const int r = n / each, row = from + (n - r * each) * 32 + l32;
+      const long off = b * s.o.bs + (static_cast<long>(gidx) * s.rep + r) * s.o.hs;
+      u32x4 gf[KK];
+      row_frags<D>(gy + off, s.o.rs, row, T, lg, gf);
+      const float del = flash_row_delta<D>(gf, out + off, resid ? resid + off : nullptr, s.o.rs, row, T, lg);
+      if (lg == 0 && row < T) own[r * (T - from) + row - from] = del;
+    }
+    __syncthreads();
+  }
   arrive(0);
   meet();
   aim(steps > 1);
@@ -1118,31 +1158,24 @@ __device__ __forceinline__ void flash_dq_tile(const char* k_rows, const char* v_
   }
 }
 
+// A workgroup's blocks of the dQ pass: a late query block, then its mirror image from the front (see the forward kernel). `lds` holds
+// flash_dq_lds bytes; the mean key behind the tiles.
 template <int D, typename TO, bool WIN, int GROUPS>
-__global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_bwd_dq_kernel(
+__device__ __forceinline__ void flash_dq_blocks(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
     const unsigned short* __restrict__ out, const unsigned short* __restrict__ resid, const float* __restrict__ lse,
-    float* __restrict__ delta, const unsigned short* __restrict__ gy, TO* __restrict__ gq, FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
+    float* __restrict__ delta, const unsigned short* __restrict__ gy, TO* __restrict__ gq, const FlashShape& s, char* flash_lds, int pair, long plane,
+    OmxFaultWord* fault, unsigned long long tag) {
   constexpr int NT = FT / GROUPS, ROW_WAVES = 4 / GROUPS, ROWS = 32 * ROW_WAVES;
   constexpr int KK = D / 16, MT = D / 32, NL = 8 * D / NT;
-  // Two key / value tile pairs (per group), as in the forward: one barrier per tile.
-  __shared__ __attribute__((aligned(16))) char flash_lds[GROUPS * 4 * ftile(D)];
-  __shared__ __attribute__((aligned(16))) float mean_key[D];
   const int lane = threadIdx.x & 63, l32 = lane & 31, lg = lane >> 5;
   const int group = GROUPS == 1 ? 0 : wave_index() / ROW_WAVES, wave = GROUPS == 1 ? wave_index() : wave_index() % ROW_WAVES;
+  // Two key / value tile pairs (per group), as in the forward: one barrier per tile.
   char* const smem = flash_lds + group * (4 * ftile(D));
+  float* const mean_key = reinterpret_cast<float*>(flash_lds + GROUPS * 4 * ftile(D));
   const int T = s.time;
   const TileFetch<D, NT> fetch(s.kv.rs, T);
-  // A late query block, then its mirror image from the front (see the forward kernel).
   const int q_blocks = (T + ROWS - 1) / ROWS;
-  int pair;
-  long plane;
-  if (s.q_single) {  // block rank (0 = the last, heaviest block) in the high part of the index
-    pair = static_cast<int>(blockIdx.x) / (s.batch * s.heads);
-    plane = static_cast<int>(blockIdx.x) % (s.batch * s.heads);
-  } else {
-    flash_block_of((q_blocks + 1) / 2, s.batch * s.heads, &pair, &plane);
-  }
   for (int pass = 0; pass < (s.q_single ? 1 : 2); ++pass) {
     const int qb = pass == 0 ? q_blocks - 1 - pair : pair;
     if (pass == 1 && qb >= q_blocks - 1 - pair) break;
@@ -1161,30 +1194,13 @@ __global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_bwd_dq_kerne
     // is off by 2^-9 of |dO| |O|, which a component shared by all value rows (and by all key rows,
     // in dQ = dS K) turns into a multiple of the gradient itself. With the saved rounding residual
     // of the output the mismatch drops to 2^-17.
-    float row_del = 0.0f;
-    {
-      auto dot_rows = [&](const unsigned short* plane) {
-        u32x4 of[KK];
-        row_frags<D>(plane + b * s.o.bs + h * s.o.hs, s.o.rs, q_row, T, lg, of);
-        float sum = 0.0f;
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-          const unsigned int gw[4] = {gf[kk].x, gf[kk].y, gf[kk].z, gf[kk].w};
-          const unsigned int ow[4] = {of[kk].x, of[kk].y, of[kk].z, of[kk].w};
-#pragma unroll
-          for (int w = 0; w < 4; ++w) sum = dot_pairs(gw[w], ow[w], sum);
-        }
-        return sum;
-      };
-      row_del = dot_rows(out);
-      if (resid) row_del += dot_rows(resid);
-      row_del = halves_sum(row_del);
-    }
+    const long o_off = b * s.o.bs + h * s.o.hs;
+    const float row_del = flash_row_delta<D>(gf, out + o_off, resid ? resid + o_off : nullptr, s.o.rs, q_row, T, lg);
     float row_lse = 0.0f;
     bool bad = false;
     if (q_row < T) {
       row_lse = lse[plane * T + q_row];
-      if (lg == 0 && group == 0) delta[plane * T + q_row] = row_del;
+      if (delta && lg == 0 && group == 0) delta[plane * T + q_row] = row_del;
       bad |= !(dev_finite(row_lse) && dev_finite(row_del));
     }
     const float neg_lse = -row_lse * LOG2E;
@@ -1305,6 +1321,46 @@ __global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_bwd_dq_kerne
     bad |= store_transposed_acc<D, TO>(gq + b * s.q.bs + h * s.q.hs, s.q.rs, q_row, T, lg, dq, s.scale);
     if (bad) dev_raise_fault(fault, tag);
   }  // pass
+}
+
+template <int D, typename TO, bool WIN, int GROUPS>
+__global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_bwd_dq_kernel(
+    const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
+    const unsigned short* __restrict__ out, const unsigned short* __restrict__ resid, const float* __restrict__ lse,
+    float* __restrict__ delta, const unsigned short* __restrict__ gy, TO* __restrict__ gq, FlashShape s, OmxFaultWord* fault, unsigned long long tag) {
+  __shared__ __attribute__((aligned(16))) char flash_lds[flash_dq_lds(D, GROUPS)];
+  int pair;
+  long plane;
+  if (s.q_single) {  // block rank (0 = the last, heaviest block) in the high part of the index
+    pair = static_cast<int>(blockIdx.x) / (s.batch * s.heads);
+    plane = static_cast<int>(blockIdx.x) % (s.batch * s.heads);
+  } else {
+    flash_block_of((s.time + 256 / GROUPS - 1) / (256 / GROUPS), s.batch * s.heads, &pair, &plane);
+  }
+  flash_dq_blocks<D, TO, WIN, GROUPS>(q, k, v, out, resid, lse, delta, gy, gq, s, flash_lds, pair, plane, fault, tag);
+}
+
+// Both passes in one launch (flash_together says when): the key side's workgroups, which form delta themselves, then the dQ pass's. Every
+// block is a workgroup's of its own (s.q_single, s.kv_single). The dQ pass's windowed form also serves calls without a window.
+template <int D, typename TO, int GROUPS>
+__global__ __launch_bounds__(FT, flash_dkv_waves(D, GROUPS)) void flash_bwd_kernel(
+    const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, const unsigned short* __restrict__ v,
+    const unsigned short* __restrict__ out, const unsigned short* __restrict__ resid, const float* __restrict__ lse,
+    const unsigned short* __restrict__ gy, TO* __restrict__ gq, TO* __restrict__ gk, TO* __restrict__ gv, FlashShape s, OmxFaultWord* fault,
+    unsigned long long tag) {
+  constexpr int KEY_LDS = GROUPS * 2 * flash_dkv_set(D) + FLASH_OWN_ROWS * 4;
+  __shared__ __attribute__((aligned(256))) char lds[KEY_LDS > flash_dq_lds(D, GROUPS) ? KEY_LDS : flash_dq_lds(D, GROUPS)];
+  const int blocks = (s.time + 128 / GROUPS - 1) / (128 / GROUPS), kv_planes = s.batch * s.kv_heads, q_planes = s.batch * s.heads;
+  const int index = static_cast<int>(blockIdx.x);
+  if (index < blocks * kv_planes) {
+    const int kb = index / kv_planes, plane = index - kb * kv_planes, b = plane / s.kv_heads;
+    const bool bad = flash_dkv_block<D, TO, GROUPS, false, true>(q, k, v, lse, nullptr, gy, gk, gv, s, lds, kb, b, plane - b * s.kv_heads, 0, out, resid,
+                                                                 reinterpret_cast<float*>(lds + GROUPS * 2 * flash_dkv_set(D)));
+    if (bad) dev_raise_fault(fault, tag);
+  } else {
+    const int n = index - blocks * kv_planes, pair = n / q_planes;
+    flash_dq_blocks<D, TO, true, GROUPS>(q, k, v, out, resid, lse, nullptr, gy, gq, s, lds, pair, n - pair * q_planes, fault, tag);
+  }
 }
 
 // `strides`: nine element strides (row, head, batch of q; of k / v; of out), or null for
@@ -1477,6 +1533,71 @@ FlashKeyPlan flash_key_plan(omx_ctx* ctx, const FlashShape& s, int dim) {
   return plan;
 }
 
+// Whether the two passes of the backward share a launch, and then how many groups of waves take a block's tiles (0: two launches). Each
+// pass alone is a chain: a launch, loads, tiles of 0.9 us and more, a store; over few tiles, with places for the workgroups of both, the
+// chains run side by side. us of a backward, two launches / one: 8 x 12 heads x 64: 14.7 / 8.1, 96 planes x 128 18.4 / 11.3, x 256 25.2 / 21.0;
+// 2 x 8 x 512 22.9 / 16.9; 10 x 3 x 320 23.1 / 16.3; head_dim 128: 4 x 8 x 64 20.8 / 12.0, x 256 30.8 / 20.2, x 640 59 / 43. Groups by an
+// estimate of the form of flash_key_plan's, fitted to 412 timings (rms 6 to 9 %); over 126 shapes the choice among one launch and two
+// takes 0.7 % more than the best of all, 22 % less than two launches. Left to two: many workgroups, where the dQ pass alone has three
+// per compute unit (16 x 16 x 256: 32.6 / 36.3; head_dim 128, 13 x 12 x 256: 53 / 54, x 512 101 / 131), and many query heads over a KV
+// head, whose tiles one workgroup walks (6 x 12 over 3 x 256: 29.1 / 29.7; the parts of flash_key_plan take those).
+// Gradients over what the other pass still reads take two launches too, as they always could.
+int flash_together(omx_ctx* ctx, const FlashShape& s, int dim, const void* q, const void* k, const void* v, const void* out, const void* resid,
+                   const void* gy, const void* gq, const void* gk, const void* gv) {
+  if (ctx->attention_together == 0 || static_cast<long>(s.rep) * s.time > FLASH_OWN_ROWS) return 0;
+  const long units = ctx->cu_count > 0 ? ctx->cu_count : 256, planes = static_cast<long>(s.batch) * (s.kv_heads + s.heads);
+  if (planes * ((s.time + 31) / 32) > 0x7fffffffl) return 0;
+  const int tiles = flash_tiles(s);
+  if (ctx->attention_together < 0) {
+    if (ctx->flash_schedule != 0) return 0;  // (a forced cut is that of two launches)
+    const long ones = (s.time + 127) / 128 * planes, fours = (s.time + 31) / 32 * planes;
+    const bool few = dim == 64 ? (tiles <= 13 && 8 * ones <= 25 * units && (s.rep == 1 || s.rep * tiles <= 16)) || (s.rep == 1 && fours <= units)
+                               : (ones <= units || (tiles >= 5 && 8 * ones <= 15 * units)) && (s.rep == 1 || s.rep * tiles <= 12);
+    if (!few) return 0;
+  }
+  struct Range {
+    const char *first, *end;
+  };
+  auto range = [&](const void* p, const FlashStrides& t, long n) {
+    const char* first = static_cast<const char*>(p);
+    return Range{first, first + 2 * ((s.batch - 1) * t.bs + (n - 1) * t.hs + (s.time - 1) * t.rs + dim)};
+  };
+  const Range read[] = {range(q, s.q, s.heads), range(k, s.kv, s.kv_heads), range(v, s.kv, s.kv_heads), range(out, s.o, s.heads),
+                        range(gy, s.o, s.heads), range(resid ? resid : out, s.o, s.heads)};
+  const Range written[] = {range(gq, s.q, s.heads), range(gk, s.kv, s.kv_heads), range(gv, s.kv, s.kv_heads)};
+  for (const Range& r : read)
+    for (const Range& w : written)
+      if (r.first < w.end && w.first < r.end) return 0;
+  const int most = dim == 64 ? 4 : 2;
+  if (ctx->flash_schedule != 0) return ctx->flash_schedule < 3 ? 1 : std::min(most, ctx->flash_schedule == 3 ? 2 : 4);
+  struct Fit {
+    double first, step, work, each;  // us: of a workgroup, of a tile on its way; of a unit's tiles, of a unit's workgroups
+  };
+  const Fit fits[2][3] = {{{6.1, 2.1, 1.26, 4.0}, {7.1, 2.4, 1.15, 4.8}, {7.7, 3.0, 3.25, 4.5}}, {{9.2, 3.15, 2.9, 10.0}, {9.6, 4.3, 2.7, 11.0}, {}}};
+  int best = 1;
+  double least = 1e30;
+  for (int g = 1, shift = 0; g <= most; g *= 2, ++shift) {
+    const int rows = 128 / g, blocks = (s.time + rows - 1) / rows;
+    const Fit& f = fits[dim == 128][shift];
+    long walk = 0, all = 0;
+    for (int n = 0; n < blocks; ++n) {
+      const int first = n * rows, last = std::min(s.time - 1, first + rows - 1);
+      const int until = s.window > 0 ? std::min(s.time - 1l, last + s.window - 1l) : s.time - 1, from = s.window > 0 ? std::max(0, first + 1 - s.window) : 0;
+      const long keys = (static_cast<long>(s.rep) * (until / 64 - first / 64 + 1) + g - 1) / g, queries = (last / 64 - from / 64 + g) / g;
+      all += s.batch * (s.kv_heads * keys + s.heads * queries);
+      walk = std::max(walk, keys);
+    }
+    const double one = f.first + f.step * static_cast<double>(walk);
+    const double work = (f.work * static_cast<double>(all) + f.each * static_cast<double>(blocks * planes)) / static_cast<double>(units);
+    const double us = one * one + work * work;
+    if (us < least) {
+      least = us;
+      best = g;
+    }
+  }
+  return best;
+}
+
 template <int D>
 void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short* k, const unsigned short* v,
                      const unsigned short* out, const unsigned short* resid, const float* lse, float* delta,
@@ -1489,6 +1610,18 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
   dim3 block(FT);
   const unsigned pairs = static_cast<unsigned>((s.time + 127) / 128 + 1) / 2;  // two 128-row blocks per workgroup
   const unsigned kv_planes = static_cast<unsigned>(s.batch * s.kv_heads), q_planes = static_cast<unsigned>(s.batch * s.heads);
+  const int together = grad_dtype == OMX_BF16 ? flash_together(ctx, s, D, q, k, v, out, resid, gy, gq, gk, gv) : 0;
+  if (together) {
+    const unsigned rows = 128 / together, blocks = (static_cast<unsigned>(s.time) + rows - 1) / rows;
+    s.q_single = s.kv_single = 1;
+    if (s.window == 0) s.window = s.time;  // (the same pairs)
+    for_groups<D>(together, [&](auto count) {
+      omx_launch_timed(ctx, flash_bwd_kernel<D, unsigned short, decltype(count)::value>, dim3(blocks * (kv_planes + q_planes)), block, 0, timer.start(),
+                       timer.stop(), q, k, v, out, resid, lse, gy, static_cast<unsigned short*>(gq), static_cast<unsigned short*>(gk),
+                       static_cast<unsigned short*>(gv), s, ctx->fault, tag);
+    });
+    return;
+  }
   const int tiles = flash_tiles(s);
   const int q_groups = flash_groups(ctx, q_planes, s.time, tiles, s.window > 0, D);
   const FlashKeyPlan plan = flash_key_plan(ctx, s, D);

@@ -134,7 +134,7 @@ struct omx_ctx {
   int gemm_thin = 1;         // outputs of at most 64 columns over many rows take gemm_thin_kernel
   int flash_schedule = 0;     // 0: by the chip's workgroup places; 1: one 128-row block per workgroup; 2: mirrored pairs
   int flash_kv_parts = 0;     // workgroups that share a key block's query tiles: 0: by estimate; 1..64: always that many
-  int attention_together = -1;  // f32 attention backward in one launch: -1: by rule; 0: never; 1: wherever it can
+  int attention_together = -1;  // attention backward in one launch: -1: by rule; 0: never; 1: wherever it can
   int kv_attention_mode = 0;  // 1: cached attention always takes the LDS-tiled kernel
   int adamw_trust = 1;        // 0: omx_adamw_step_bounded always runs its checking pass
   int ce_fused = 1;           // 0: linear-CE always takes the separate statistics and gradient kernels

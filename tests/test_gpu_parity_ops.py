@@ -555,6 +555,39 @@ def test_f32_attention_backward_in_one_launch_has_the_bits_of_two(be, shape, hkv
         be.set_option("attention_together", -1)
 
 
+@pytest.mark.parametrize("schedule", [1, 3, 4])
+@pytest.mark.parametrize("shape,hkv,window", [((1, 1, 1, 64), 1, None), ((2, 2, 63, 64), 2, None), ((1, 4, 65, 128), 2, None), ((2, 8, 128, 64), 2, 33),
+                                              ((3, 5, 129, 64), 5, None), ((1, 2, 200, 128), 2, 50), ((2, 3, 333, 64), 3, 64), ((1, 1, 1024, 64), 1, None),
+                                              ((1, 1, 1000, 128), 1, 300), ((1, 16, 64, 64), 1, None)])
+def test_bf16_attention_backward_in_one_launch_has_the_bits_of_two(be, shape, hkv, window, schedule):
+    """Both passes of the bf16 backward in one launch on one, two and four groups of waves, the key side's row terms formed there: every
+    bit of two launches, last tiles and row blocks past the end, groups of heads and windows among them. Gradients in place of
+    keys and values, which the other pass reads, take two."""
+    from ojas_amd.backend import BF16, _native
+
+    b, h, t, d = shape
+    print(f"bf16 backward together {shape} {hkv} {window} {schedule}", flush=True)
+    rng = np.random.default_rng(t)
+    x = [be.upload(rng.normal(size=(b, n, t, d)).astype(np.float32), BF16) for n in (h, hkv, hkv, h)]
+    y, lse = be.causal_sdpa_forward(*x[:3], window, BF16)
+    got = {}
+    try:
+        be.set_option("flash_schedule", schedule)
+        for together in (0, 1):
+            be.set_option("attention_together", together)
+            got[together] = [be.download(g) for g in be.causal_sdpa_backward(*x[:3], y, lse, x[3], window, BF16)]
+        for two, one in zip(got[0], got[1]):
+            np.testing.assert_array_equal(one, two)
+        gq = be.empty(shape, BF16)
+        _native.omx_causal_sdpa_backward(be._context, x[0], x[1], x[2], y, lse, x[3], BF16, BF16, BF16, gq, x[1], x[2], BF16, b, h, hkv, t, d,
+                                         window or 0)
+        for g, e in zip((gq, x[1], x[2]), got[0]):
+            np.testing.assert_array_equal(be.download(g), e)
+    finally:
+        be.set_option("attention_together", -1)
+        be.set_option("flash_schedule", 0)
+
+
 def test_f32_attention_backward_of_more_workgroups_than_an_axis_holds(be):
     """65535 planes of 2064 positions: each pass has 2^23 workgroups and more, both together over 2^24, which are 2^32 threads (70 GB of
     tensors, all zeros but a gradient of ones: every weight is 1, so a value's gradient counts the queries that see it)."""
