@@ -674,15 +674,18 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   // own kernel, which neither tiles the output nor splits K across launches.
   const bool thin = operand_dtype == OMX_BF16 && !low_rank && ctx->gemm_thin && !(epi && epi->mode != OMX_EPI_NONE) &&
                     omx_gemm_thin_eligible(g, a_km, b_km);
+  // A few heads' weight gradients, whose rows the direct-to-LDS kernels cannot read.
+  const bool heads = operand_dtype == OMX_BF16 && !low_rank && ctx->gemm_thin && ctx->gemm_dma_mode == 1 && !(epi && epi->mode != OMX_EPI_NONE) && !g.a_vec &&
+                     omx_gemm_heads_eligible(g, a_km, b_km);
   // Few rows (a decoder's linear layers): K shared between a workgroup's waves, no tile of 128 rows.
   const double skinny_us = operand_dtype == OMX_BF16 && !thin && !low_rank && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
                                ? omx_gemm_skinny_us(ctx, g, a_km, b_km, epi && epi->mode != OMX_EPI_NONE) : -1.0;
-  bool skinny = skinny_us >= 0.0;
+  bool skinny = skinny_us >= 0.0 && !heads;
   int frag32 = -1, dma32 = -1;
   if (operand_dtype == OMX_F32 && ctx->gemm_dma_mode == 1 && !(epi && epi->mode != OMX_EPI_NONE))
     f32_tile(ctx, g, a_km, b_km, &frag32, &dma32);
   int dma_variant = -1, small_splits = 0;
-  if (!thin && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) {
+  if (!thin && !heads && operand_dtype == OMX_BF16 && omx_gemm_dma_eligible(g, a_km, b_km, !(epi && epi->mode != OMX_EPI_NONE))) {
     const int mode = ctx->gemm_dma_mode;
     if (mode == 1 && ctx->gemm_forced_tiling >= 0) {
       dma_variant = ctx->gemm_forced_tiling;
@@ -926,9 +929,11 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     }
     if (small_splits > 0) splits = small_splits;  // chosen with the tiling
     else if (dma_variant == 7 || dma_variant == 8) splits = 1;
-    g.ksteps_per_split = (ksteps + splits - 1) / splits;
+    if (heads) splits = omx_gemm_heads_splits(g);
+    const int steps = heads ? (g.K + 31) / 32 : ksteps;  // (of 32 rows there)
+    g.ksteps_per_split = (steps + splits - 1) / splits;
     if (dma_variant >= 9) g.ksteps_per_split += g.ksteps_per_split & 1;  // its K loop takes steps in pairs
-    g.splits = (ksteps + g.ksteps_per_split - 1) / g.ksteps_per_split;
+    g.splits = (steps + g.ksteps_per_split - 1) / g.ksteps_per_split;
     g.partial = nullptr;
     if (g.splits > 1) {
       void* ws = nullptr;
@@ -1024,8 +1029,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     rc = omx_gemm_frag32_launch(ctx, g, a_km, b_km, frag32);
   } else if (skinny) {
     rc = omx_gemm_skinny_launch(ctx, g);
-  } else if (dma_variant >= 0) {
-    rc = omx_gemm_dma_launch(ctx, g, a_km, b_km, dma_variant);
+  } else if (dma_variant >= 0 || heads) {
+    rc = heads ? omx_gemm_heads_launch(ctx, g) : omx_gemm_dma_launch(ctx, g, a_km, b_km, dma_variant);
     if (rc == OMX_OK && g.splits > 1) {
       long elems = static_cast<long>(g.M) * g.N;
       unsigned blocks = static_cast<unsigned>(std::min<long>((elems + 255) / 256, 4096));

@@ -388,6 +388,11 @@ int32_t omx_gemm_dma_launch(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_k
 bool omx_gemm_thin_eligible(const GemmArgs& g, bool a_km, bool b_km);
 int32_t omx_gemm_thin_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km);
 
+// bf16 kernel for outputs of at most 16 rows from two k-major operands, A's pitch any (no accumulation).
+bool omx_gemm_heads_eligible(const GemmArgs& g, bool a_km, bool b_km);
+int omx_gemm_heads_splits(const GemmArgs& g);
+int32_t omx_gemm_heads_launch(omx_ctx* ctx, const GemmArgs& g);
+
 // bf16 kernel for products of few rows or few outputs, both operands k-contiguous, K a multiple of 32.
 double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, bool activation);
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);

@@ -96,6 +96,7 @@ struct onano {
   void *g_v0 = nullptr;                  // [N, KV D] AD: what the later blocks' blends send to block 0's v
   void *g_qkv = nullptr, *g_qkv_lin = nullptr, *gqkv_all = nullptr;  // fused projection: gradients [N, P3] AD
   void* gz_all = nullptr;  // the gates' pre-activation gradients [layers][N, heads] AD (deferred weight gradients)
+  uint64_t gz_stride = 0;  // elements from a layer's to the next one's: a strided batch wants its products whole 16 bytes apart
   float* v0_acc = nullptr;               // the same as g_v0 in f32 (fused projection)
   void *gqp = nullptr, *gkp = nullptr, *gvp = nullptr, *gap_p = nullptr;  // permuted gradients (row kernels)
   void *gy16 = nullptr, *ghf = nullptr;
@@ -309,16 +310,16 @@ int32_t backward(onano* t, float loss_seed) {
     const bool gate_f32 = t->keep_f32 && t->flash;
     const int32_t GD = gate_f32 ? OMX_F32 : AD;
     TRY(omx_linear_backward(ctx, A.y, t->w(t->li(l, WO)), gy, AD, t->gyy, GD, gw(WO), OMX_F32, N, qd, d));
-    const bool gz_waits = defer && t->gz_all;  // the gate's weight gradient waits for the batched product below
+    const bool gz_waits = defer;  // the gate's weight gradient waits for the batched product below
     if (gate_f32)
       TRY(omx_per_head_sigmoid_gate_sum_backward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap, A.apr, t->gyy, A.gates,
                                                  gz_waits && t->fused_qkv ? nullptr : t->gh, OMX_F32,
-                                                 gz_waits ? nullptr : t->g(t->li(l, GATE_W)), gz_waits ? slice(t->gz_all, l, N * H) : nullptr,
+                                                 gz_waits ? nullptr : t->g(t->li(l, GATE_W)), gz_waits ? slice(t->gz_all, l, t->gz_stride) : nullptr,
                                                  t->g(t->li(l, GATE_B)), t->gap, AD, N, d, H, D));
     else if (gz_waits)
       TRY(omx_per_head_sigmoid_gate_backward_deferred(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap,
                                                       AD, t->gyy, AD, A.gates, t->fused_qkv ? nullptr : t->gh, OMX_F32,
-                                                      slice(t->gz_all, l, N * H),
+                                                      slice(t->gz_all, l, t->gz_stride),
                                                       t->g(t->li(l, GATE_B)), t->gap, AD, N, d, H, D));
     else
       TRY(omx_per_head_sigmoid_gate_backward(ctx, A.h, t->w(t->li(l, GATE_W)), AD, t->w32(t->li(l, GATE_B)), A.ap, AD,
@@ -343,8 +344,8 @@ int32_t backward(onano* t, float loss_seed) {
       if (!blends) TRY(omx_fill_zero(ctx, t->g(t->li(0, LAMBDA)), 4));
       // One product for the three projections: their input gradients add in its f32 accumulators.
       TRY(omx_linear_backward(ctx, A.h, t->w(t->li(l, WQ)), g_lin, AD, t->t_a, AD, gw(WQ), OMX_F32, N, d, P3));
-      if (defer && t->gz_all)  // the gate's input gradient, left out above, joins here in one pass
-        TRY(omx_per_head_sigmoid_gate_input_grad_add(ctx, slice(t->gz_all, l, N * H), t->w(t->li(l, GATE_W)), AD, t->t_a,
+      if (gz_waits)  // the gate's input gradient, left out above, joins here in one pass
+        TRY(omx_per_head_sigmoid_gate_input_grad_add(ctx, slice(t->gz_all, l, t->gz_stride), t->w(t->li(l, GATE_W)), AD, t->t_a,
                                                      AD, t->gh, N, d, H));
       else
         TRY(omx_residual_add(ctx, t->gh, OMX_F32, t->t_a, AD, t->gh, OMX_F32, N * d));
@@ -415,9 +416,8 @@ int32_t backward(onano* t, float loss_seed) {
                                  layers, N * p.out, N * p.in, per_layer));
     }
     // The gates' weight gradients: heads x d each over all tokens, every block in one launch.
-    if (t->gz_all)
-      TRY(omx_gemm_strided_batch(ctx, t->gz_all, 1, H, t->h_all, d, 1, AD, t->g(t->li(0, GATE_W)), OMX_F32, H, N, d, 0, layers,
-                               N * H, N * d, per_layer));
+    TRY(omx_gemm_strided_batch(ctx, t->gz_all, 1, H, t->h_all, d, 1, AD, t->g(t->li(0, GATE_W)), OMX_F32, H, N, d, 0, layers, t->gz_stride, N * d,
+                               per_layer));
   }
   // The tied table: the head's gradient first, then the embedding's rows.
   // The tied table: the gather's gradient joins the head's where it lies, row by named row.
@@ -555,8 +555,8 @@ int32_t onano_create(omx_ctx* ctx, const onano_config* config, onano** out) {
     CREATE_TRY(alloc_act(t, L * N * d, &t->gyd_all));
     CREATE_TRY(alloc_act(t, L * 2 * N * Hd, &t->ggu_all));
     CREATE_TRY(alloc_act(t, L * N * d, &t->gyo_all));
-    // (a strided batch wants its products 16 bytes apart at least)
-    if ((N * c.heads * t->asz) % 16 == 0) CREATE_TRY(alloc_act(t, L * N * c.heads, &t->gz_all));
+    t->gz_stride = (N * c.heads + 7) / 8 * 8;
+    CREATE_TRY(alloc_act(t, L * t->gz_stride, &t->gz_all));
     if (t->fused_qkv) {
       CREATE_TRY(alloc_act(t, L * N * (qd + 2 * kd), &t->gqkv_all));
     } else {

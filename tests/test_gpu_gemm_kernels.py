@@ -881,3 +881,33 @@ def test_gates_and_ups_of_one_product_have_the_bits_of_two_calls(be, rows, kin, 
     finally:
         be.set_option("gemm_dma", 1)
         be.set_option("q8_widen", -1)
+
+
+@pytest.mark.parametrize("m,k,n,lda,count", [(1, 1, 8, 1, 1), (5, 31, 64, 5, 3), (10, 282, 640, 10, 2), (12, 33, 72, 12, 1), (16, 1023, 264, 17, 2), (13, 1024, 256, 13, 1),
+                                             (12, 1025, 768, 12, 3), (3, 2049, 8, 9, 1), (12, 8200, 328, 12, 2), (15, 20000, 128, 15, 1)])
+@pytest.mark.parametrize("bf16_out", [False, True])
+def test_weight_gradients_of_a_few_heads(be, m, k, n, lda, count, bf16_out):
+    """`gemm_heads_kernel`: at most 16 rows from two operands by rows of the reduction, A's pitch any; one share of the rows and several,
+    partial last steps and column blocks. f32 sums of exact products: within k roundings of the terms' size."""
+    from ojas_amd.backend import BF16, F32
+
+    rng = np.random.default_rng(m + k + n)
+    stride_a, stride_b = -(-k * lda // 8) * 8, k * n
+    a = np.zeros((count, stride_a), np.float32)
+    for i in range(count):
+        a[i, :k * lda] = rng.normal(0, 1, k * lda)
+    b = rng.normal(0, 1, (count, k, n)).astype(np.float32)
+    da, db = be.upload(a, BF16), be.upload(b, BF16)
+    if count == 1:
+        got = be.gemm(da, (1, lda), db, (n, 1), m, k, n, BF16 if bf16_out else F32)
+    else:
+        stride_c = -(-m * n // 8) * 8
+        got = be.gemm_strided_batch(da, (1, lda), db, (n, 1), m, k, n, count, (stride_a, stride_b, stride_c), BF16 if bf16_out else F32)
+    got = be.download_f32(got).reshape(-1)
+    ar, br = be.download_f32(da).astype(np.float64), be.download_f32(db).astype(np.float64).reshape(count, k, n)
+    for i in range(count):
+        ai = ar.reshape(count, stride_a)[i, :k * lda].reshape(k, lda)[:, :m]
+        want, size = ai.T @ br[i], np.abs(ai).T @ np.abs(br[i])
+        at = 0 if count == 1 else i * stride_c
+        part = got[at:at + m * n].reshape(m, n)
+        assert np.all(np.abs(part - want) <= size * k * 2.0**-24 + (np.abs(want) * 2.0**-8 if bf16_out else 0) + 1e-30)
