@@ -754,9 +754,11 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * "gemm_f32": -1 = f32 products take the tile with the least estimated time (default), 0 .. 4 = always the register-fragment
  * kernel's 16 x 16 / 16 x 32 / 32 x 32 / 64 x 32 / 64 x 64 tile, 5 .. 8 = the direct-to-LDS kernel's 64 x 64 / 64 x 32 / 64 x 32 by
  * two wave groups / 32 x 32 by four, wherever the operands fit it, 9 = the register-staged kernel.
+ * "gemm_skinny_km": -1 = bf16 products of few rows with a B by rows of K share K between eight waves where that is estimated to be ahead
+ * (default), 0 = never, 1 or 2 = wherever the operands fit it, on workgroups of 16 or 32 rows.
  * "gemm_thin": 0 = bf16 products with at most 64 output columns over 1024 rows or
  * more go through the tiled kernels and their split-K reduce instead of the one-pass kernel for
- * thin outputs (default 1). "q8_widen": int8 products over a widened copy of the weight in scratch: -1 = where
+ * thin outputs, and those of at most 16 rows by rows of K too (default 1). "q8_widen": int8 products over a widened copy of the weight in scratch: -1 = where
  * that is estimated to be ahead (default), 0 = never, 1 = wherever they can. "gemm_row_split": 0 = a product on 256x256 tiles whose last round
  * of tiles fills under 2/5 of the compute units is not cut into two launches by rows (default 1:
  * the rows of the whole rounds keep the tiling, the rest choose their own). "kv_attention": 0 = choose by head_dim (default), 1 = always the

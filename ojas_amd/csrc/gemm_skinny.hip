@@ -155,6 +155,113 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows4_kernel(GemmArgs g) {
   }
 }
 
+// The same with B by rows of K (an input gradient's weights): 16 MB rows by 64 columns a workgroup, whose waves take runs of 32-row steps
+// of K. B comes in pieces of a row and turns in LDS of the wave's own (144-byte rows: the four rows of a transposing read lie in
+// different banks), SKINNY_KM_CHUNK steps in flight together, no barrier before the waves' sums meet.
+typedef short short4_s __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2_s __attribute__((ext_vector_type(2)));
+constexpr int KM_PITCH = 144, KM_CHUNK = 2;
+template <int MB, int WAVES>
+constexpr int km_lds() {
+  return WAVES * KM_CHUNK * 32 * KM_PITCH > WAVES * MB * 4096 ? WAVES * KM_CHUNK * 32 * KM_PITCH : WAVES * MB * 4096;
+}
+template <int MB, int WAVES, bool PLAIN>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_km_kernel(GemmArgs g) {
+  extern __shared__ __attribute__((aligned(16))) char km_smem[];
+  gemm_select_batch(g, blockIdx.z);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int l16 = lane & 15, kg = lane >> 4, piece = lane & 7, krow = lane >> 3;
+  const int row0 = blockIdx.y * (16 * MB), col0 = blockIdx.x * 64;
+  // Rows and columns past the end are read from the last ones and never stored.
+  const unsigned short* a[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) a[m] = static_cast<const unsigned short*>(g.a) + static_cast<long>(min(row0 + m * 16 + l16, g.M - 1)) * g.lda + kg * 8;
+  const unsigned short* const b = static_cast<const unsigned short*>(g.b) + min(col0 + piece * 8, g.N - 8) + static_cast<long>(krow) * g.ldb;
+  char* const own = km_smem + wave * (KM_CHUNK * 32 * KM_PITCH);
+  floatx4_s acc[MB][4];
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[m][n] = floatx4_s{0.0f, 0.0f, 0.0f, 0.0f};
+  const int steps = g.K / 32, s_end = steps * (wave + 1) / WAVES;
+  u32x4_s bf[KM_CHUNK][4], af[KM_CHUNK][MB];
+  auto fetch = [&](int s0) {
+#pragma unroll
+    for (int s = 0; s < KM_CHUNK; ++s)
+      if (s0 + s < s_end) {  // uniform over the wave
+        const long k = static_cast<long>(s0 + s) * 32;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bf[s][i] = *reinterpret_cast<const u32x4_s*>(b + (k + 8 * i) * g.ldb);
+#pragma unroll
+        for (int m = 0; m < MB; ++m) af[s][m] = *reinterpret_cast<const u32x4_s*>(a[m] + k);
+      }
+  };
+  int s0 = steps * wave / WAVES;
+  fetch(s0);
+  for (; s0 < s_end; s0 += KM_CHUNK) {
+    const int live = min(KM_CHUNK, s_end - s0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the previous rows have been read
+    u32x4_s am[KM_CHUNK][MB];
+#pragma unroll
+    for (int s = 0; s < KM_CHUNK; ++s)
+      if (s < live) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4_s*>(own + (s * 32 + i * 8 + krow) * KM_PITCH + piece * 16) = bf[s][i];
+#pragma unroll
+        for (int m = 0; m < MB; ++m) am[s][m] = af[s][m];
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (s0 + KM_CHUNK < s_end) fetch(s0 + KM_CHUNK);
+#pragma unroll
+    for (int s = 0; s < KM_CHUNK; ++s)
+      if (s < live) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          // Lane (column l16, kg) gets rows 8 kg .. 8 kg + 7 of column n * 16 + l16.
+          typedef short4_s __attribute__((address_space(3))) * lds_ptr;
+          const char* p = own + (s * 32 + kg * 8 + (l16 >> 2)) * KM_PITCH + n * 32 + (l16 & 3) * 8;
+          const u32x2_s lo = __builtin_bit_cast(u32x2_s, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p)));
+          const u32x2_s hi = __builtin_bit_cast(u32x2_s, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 4 * KM_PITCH)));
+          const u32x4_s w = u32x4_s{lo.x, lo.y, hi.x, hi.y};
+#pragma unroll
+          for (int m = 0; m < MB; ++m)
+            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_s, w), __builtin_bit_cast(bf16x8_s, am[s][m]), acc[m][n], 0, 0, 0);
+        }
+      }
+  }
+  __syncthreads();  // the steps' LDS has been read
+  // acc[m][n][v] is row m * 16 + l16, column n * 16 + 4 * (lane / 16) + v of this wave's share of K.
+  float* const red = reinterpret_cast<float*>(km_smem);
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[((wave * (MB * 4) + m * 4 + n) * 4 + v) * 64 + lane] = acc[m][n][v];
+  __syncthreads();
+  bool bad = false;
+  for (int blk = wave; blk < MB * 4; blk += WAVES) {
+    const int row = row0 + blk / 4 * 16 + l16, col = col0 + blk % 4 * 16 + kg * 4;
+    float x[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      float part[WAVES];
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) part[w] = red[((w * (MB * 4) + blk) * 4 + v) * 64 + lane];
+#pragma unroll
+      for (int span = 1; span < WAVES; span *= 2)
+#pragma unroll
+        for (int w = 0; w < WAVES; w += 2 * span) part[w] += part[w + span];
+      x[v] = part[0];
+    }
+    if (row < g.M && col < g.N)
+      bad |= PLAIN ? gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3]) : gemm_store4_epi(g, 0, row, col, x[0], x[1], x[2], x[3]);
+  }
+  if (bad) dev_raise_fault(g.fault, g.tag);
+}
+
 struct SkinnyTile {
   int mb, nb;
 };
@@ -214,6 +321,18 @@ int32_t launch_rows4(omx_ctx* ctx, const GemmArgs& g) {
   return OMX_OK;
 }
 
+template <int MB>
+int32_t launch_km(omx_ctx* ctx, const GemmArgs& g) {
+  constexpr int WAVES = 8, smem = km_lds<MB, WAVES>();
+  auto kernel = g.epi == OMX_EPI_NONE ? &gemm_skinny_km_kernel<MB, WAVES, true> : &gemm_skinny_km_kernel<MB, WAVES, false>;
+  if constexpr (smem > 64 * 1024)
+    OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
+  dim3 grid(static_cast<unsigned>((g.N + 63) / 64), static_cast<unsigned>((g.M + 16 * MB - 1) / (16 * MB)), static_cast<unsigned>(g.batches));
+  omx_launch_timed(ctx, kernel, grid, dim3(WAVES * 64), smem, ctx->timing_start, ctx->timing_stop, g);
+  OMX_LAUNCH_CHECK(ctx, "gemm_skinny_km_kernel");
+  return OMX_OK;
+}
+
 }  // namespace
 
 // What the product takes here, in us (see skinny_tile); negative: not one for this kernel. An activation's store pass over
@@ -232,4 +351,25 @@ int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g) {
     case 2: return launch_skinny<2, 2>(ctx, g);
     default: return launch_skinny<4, 4>(ctx, g);
   }
+}
+
+// Row blocks of 16 that a workgroup of gemm_skinny_km_kernel takes, and what the product takes there, in us; negative: not one for it. One
+// block where that makes at most a workgroup per compute unit, else two where they do; a second round of workgroups is what
+// the 64 x 64 tiles gain by (400 x 2048 over 768: 7.0 there, 8.4 to 10 here). us of a call, 64 x 64 tiles / this kernel: 282 x 640 and 768
+// over 768 6.3 / 4.7, over 1280 7.9 / 6.0, over 2048 10.3 / 7.5; 64 x 1024 over 768 6.1 / 4.8; 400 x 1024 over 1280 8.4 / 7.1 (two
+// blocks); over 4096 columns of K and more the tiles' split reductions are ahead. Sums of eight short chains: errors the same or smaller.
+double omx_gemm_skinny_km_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int* mb) {
+  if (a_km || !b_km || g.K % 32 != 0 || g.K > 4096 || g.N % 8 != 0 || !g.a_vec || !g.b_vec || ctx->gemm_skinny_km == 0) return -1.0;
+  const long units = ctx->cu_count > 0 ? ctx->cu_count : 256, cols = (g.N + 63l) / 64 * g.batches;
+  if (ctx->gemm_skinny_km > 0) {  // forced (a grid's rows of workgroups are 16 bits)
+    *mb = ctx->gemm_skinny_km;
+    return g.M <= 1 << 16 ? 0.0 : -1.0;
+  }
+  *mb = (g.M + 15l) / 16 * cols <= units ? 1 : 2;
+  if (*mb == 2 && (g.M + 31l) / 32 * cols > units) return -1.0;
+  return *mb == 1 ? 2.6 + 2.2e-3 * g.K : 2.9 + 3.1e-3 * g.K;
+}
+
+int32_t omx_gemm_skinny_km_launch(omx_ctx* ctx, const GemmArgs& g, int mb) {
+  return mb == 1 ? launch_km<1>(ctx, g) : launch_km<2>(ctx, g);
 }
