@@ -754,7 +754,7 @@ int32_t omx_read_scalar_f32(omx_ctx* ctx, const void* src, float* out);
  * "gemm_f32": -1 = f32 products take the tile with the least estimated time (default), 0 .. 4 = always the register-fragment
  * kernel's 16 x 16 / 16 x 32 / 32 x 32 / 64 x 32 / 64 x 64 tile, 5 .. 8 = the direct-to-LDS kernel's 64 x 64 / 64 x 32 / 64 x 32 by
  * two wave groups / 32 x 32 by four, wherever the operands fit it, 9 = the register-staged kernel.
- * "gemm_skinny_km": -1 = bf16 products of few rows with a B by rows of K share K between eight waves where that is estimated to be ahead
+ * "gemm_skinny64": -1 = bf16 products of few rows share K between eight waves on 64 columns a workgroup where that is estimated to be ahead
  * (default), 0 = never, 1 or 2 = wherever the operands fit it, on workgroups of 16 or 32 rows.
  * "gemm_thin": 0 = bf16 products with at most 64 output columns over 1024 rows or
  * more go through the tiled kernels and their split-K reduce instead of the one-pass kernel for

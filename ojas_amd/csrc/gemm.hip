@@ -680,11 +680,10 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   // Few rows (a decoder's linear layers): K shared between a workgroup's waves, no tile of 128 rows.
   const double skinny_us = operand_dtype == OMX_BF16 && !thin && !low_rank && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
                                ? omx_gemm_skinny_us(ctx, g, a_km, b_km, epi && epi->mode != OMX_EPI_NONE) : -1.0;
-  bool skinny = skinny_us >= 0.0 && !heads;
-  int km_blocks = 0;
-  const double km_us = operand_dtype == OMX_BF16 && !thin && !low_rank && !heads && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
-                           ? omx_gemm_skinny_km_us(ctx, g, a_km, b_km, &km_blocks) : -1.0;
-  bool skinny_km = km_us >= 0.0;
+  int blocks64 = 0;
+  const double us64 = operand_dtype == OMX_BF16 && !thin && !low_rank && !heads && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
+                           ? omx_gemm_skinny64_us(ctx, g, a_km, b_km, &blocks64) : -1.0;
+  bool skinny64 = us64 >= 0.0 && (skinny_us < 0.0 || us64 < skinny_us), skinny = skinny_us >= 0.0 && !heads && !skinny64;
   int frag32 = -1, dma32 = -1;
   if (operand_dtype == OMX_F32 && ctx->gemm_dma_mode == 1 && !(epi && epi->mode != OMX_EPI_NONE))
     f32_tile(ctx, g, a_km, b_km, &frag32, &dma32);
@@ -787,8 +786,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
                                                        : before;
         auto splits_of = [&](int v) { return cheapest_split(v, g.M, g.N, g.batches, ks, limit, a_km, !plain, !g.c_vec, cus); };
         auto us_of = [&](int v, int s) { return dma_us(v, g.M, g.N, g.batches, ks, s, a_km, !plain, !g.c_vec, cus); };
-        const int first = skinny || skinny_km ? -1 : dma_variant;
-        double best = skinny ? 0.8 * skinny_us : skinny_km ? km_us : 1e30;
+        const int first = skinny || skinny64 ? -1 : dma_variant;
+        double best = skinny ? 0.8 * skinny_us : skinny64 ? us64 : 1e30;
         if (first >= 0) {
           small_splits = splits_of(first);
           best = us_of(first, small_splits);
@@ -800,12 +799,12 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
             best = us;
             dma_variant = v;
             small_splits = s;
-            skinny = skinny_km = false;
+            skinny = skinny64 = false;
           }
         }
       }
-      if (dma_variant >= 9) skinny_km = false;
-      if (skinny || skinny_km) dma_variant = -1;
+      if (dma_variant >= 9) skinny64 = false;
+      if (skinny || skinny64) dma_variant = -1;
     }
     else if (mode == 3) dma_variant = 3;
     else if (mode == 4) dma_variant = 6;
@@ -904,7 +903,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     // 108 tiles: two splits; of 2304 x 768, 324 tiles: two splits make three rounds of half the length).
     const long all_tiles = tiles * g.batches;
     const bool may_split =
-        !thin && !skinny && !skinny_km && frag32 < 0 && dma32 < 0 && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
+        !thin && !skinny && !skinny64 && frag32 < 0 && dma32 < 0 && (g.batches == 1 ? tiles < 256 : ((dma_variant < 0 && all_tiles < 512) || dma_variant >= 9));
     if (may_split && ksteps >= 4 * min_steps && !(epi && epi->mode != OMX_EPI_NONE)) {
       splits = static_cast<int>(((g.batches == 1 ? 512 : 1024) + all_tiles - 1) / all_tiles);
       if (splits > ksteps / min_steps) splits = ksteps / min_steps;
@@ -1034,8 +1033,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
     rc = omx_gemm_frag32_launch(ctx, g, a_km, b_km, frag32);
   } else if (skinny) {
     rc = omx_gemm_skinny_launch(ctx, g);
-  } else if (skinny_km) {
-    rc = omx_gemm_skinny_km_launch(ctx, g, km_blocks);
+  } else if (skinny64) {
+    rc = omx_gemm_skinny64_launch(ctx, g, b_km, blocks64);
   } else if (dma_variant >= 0 || heads) {
     rc = heads ? omx_gemm_heads_launch(ctx, g) : omx_gemm_dma_launch(ctx, g, a_km, b_km, dma_variant);
     if (rc == OMX_OK && g.splits > 1) {
@@ -1193,9 +1192,9 @@ int32_t omx_set_option(omx_ctx* ctx, const char* name, int64_t value) {
     ctx->muon_fused_sums = static_cast<int>(value);
     return OMX_OK;
   }
-  if (name && strcmp(name, "gemm_skinny_km") == 0) {
-    if (value < -1 || value > 2) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: gemm_skinny_km takes -1..2");
-    ctx->gemm_skinny_km = static_cast<int>(value);
+  if (name && strcmp(name, "gemm_skinny64") == 0) {
+    if (value < -1 || value > 2) return omx_fail(ctx, OMX_OUT_OF_RANGE, "set_option: gemm_skinny64 takes -1..2");
+    ctx->gemm_skinny64 = static_cast<int>(value);
     return OMX_OK;
   }
   if (name && strcmp(name, "muon_symmetric") == 0) {

@@ -396,9 +396,9 @@ int32_t omx_gemm_heads_launch(omx_ctx* ctx, const GemmArgs& g);
 // bf16 kernel for products of few rows or few outputs, both operands k-contiguous, K a multiple of 32.
 double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, bool activation);
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g);
-// The same with a k-major B, N a multiple of 8; `mb`: 16-row blocks of a workgroup.
-double omx_gemm_skinny_km_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int* mb);
-int32_t omx_gemm_skinny_km_launch(omx_ctx* ctx, const GemmArgs& g, int mb);
+// The same on 64 columns a workgroup, B in either layout (k-major: N a multiple of 8; else K of 64); `mb`: 16-row blocks of a workgroup.
+double omx_gemm_skinny64_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int* mb);
+int32_t omx_gemm_skinny64_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km, int mb);
 
 // f32 kernels: small outputs (gemm_frag32.hip) and direct-to-LDS loads (gemm_dma32.hip; g.K counts whole 32-column steps).
 // `_us`: what a tile is estimated to take; negative: not one for it.

@@ -155,6 +155,37 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows4_kernel(GemmArgs g) {
   }
 }
 
+// The waves' sums over 16 MB rows x 64 columns meet and go out: acc[m][n][v] is row m * 16 + lane % 16, column n * 16 + 4 * (lane / 16) + v.
+template <int MB, int WAVES, bool PLAIN>
+__device__ __forceinline__ void skinny_meet(const GemmArgs& g, const floatx4_s (&acc)[MB][4], float* red, int row0, int col0, int wave, int lane) {
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[((wave * (MB * 4) + m * 4 + n) * 4 + v) * 64 + lane] = acc[m][n][v];
+  __syncthreads();
+  bool bad = false;
+  for (int blk = wave; blk < MB * 4; blk += WAVES) {
+    const int row = row0 + blk / 4 * 16 + (lane & 15), col = col0 + blk % 4 * 16 + (lane >> 4) * 4;
+    float x[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      float part[WAVES];
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) part[w] = red[((w * (MB * 4) + blk) * 4 + v) * 64 + lane];
+#pragma unroll
+      for (int span = 1; span < WAVES; span *= 2)
+#pragma unroll
+        for (int w = 0; w < WAVES; w += 2 * span) part[w] += part[w + span];
+      x[v] = part[0];
+    }
+    if (row < g.M && col < g.N)
+      bad |= PLAIN ? gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3]) : gemm_store4_epi(g, 0, row, col, x[0], x[1], x[2], x[3]);
+  }
+  if (bad) dev_raise_fault(g.fault, g.tag);
+}
+
 // The same with B by rows of K (an input gradient's weights): 16 MB rows by 64 columns a workgroup, whose waves take runs of 32-row steps
 // of K. B comes in pieces of a row and turns in LDS of the wave's own (144-byte rows: the four rows of a transposing read lie in
 // different banks), SKINNY_KM_CHUNK steps in flight together, no barrier before the waves' sums meet.
@@ -166,7 +197,7 @@ constexpr int km_lds() {
   return WAVES * KM_CHUNK * 32 * KM_PITCH > WAVES * MB * 4096 ? WAVES * KM_CHUNK * 32 * KM_PITCH : WAVES * MB * 4096;
 }
 template <int MB, int WAVES, bool PLAIN>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_km_kernel(GemmArgs g) {
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny64_km_kernel(GemmArgs g) {
   extern __shared__ __attribute__((aligned(16))) char km_smem[];
   gemm_select_batch(g, blockIdx.z);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -232,34 +263,72 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_km_kernel(GemmArgs g) 
       }
   }
   __syncthreads();  // the steps' LDS has been read
-  // acc[m][n][v] is row m * 16 + l16, column n * 16 + 4 * (lane / 16) + v of this wave's share of K.
-  float* const red = reinterpret_cast<float*>(km_smem);
+  skinny_meet<MB, WAVES, PLAIN>(g, acc, reinterpret_cast<float*>(km_smem), row0, col0, wave, lane);
+}
+
+// The same with B's columns by K, in steps of 64: a load takes whole 128-byte lines of 8 columns, where gemm_skinny_kernel's take half
+// lines of 16, and half as many times as its 32 x 32 tiles do for their rows' share.
+template <int MB, int WAVES>
+constexpr int kc_lds() {
+  return WAVES * 64 * KM_PITCH > WAVES * MB * 4096 ? WAVES * 64 * KM_PITCH : WAVES * MB * 4096;
+}
+template <int MB, int WAVES, bool PLAIN>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny64_kc_kernel(GemmArgs g) {
+  extern __shared__ __attribute__((aligned(16))) char km_smem[];
+  gemm_select_batch(g, blockIdx.z);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int l16 = lane & 15, kg = lane >> 4, piece = lane & 7, ncol = lane >> 3;
+  const int row0 = blockIdx.y * (16 * MB), col0 = blockIdx.x * 64;
+  const unsigned short* a[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) a[m] = static_cast<const unsigned short*>(g.a) + static_cast<long>(min(row0 + m * 16 + l16, g.M - 1)) * g.lda + kg * 8;
+  const unsigned short* b[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) b[i] = static_cast<const unsigned short*>(g.b) + static_cast<long>(min(col0 + i * 8 + ncol, g.N - 1)) * g.ldb + piece * 8;
+  char* const own = km_smem + wave * (64 * KM_PITCH);
+  floatx4_s acc[MB][4];
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
+    for (int n = 0; n < 4; ++n) acc[m][n] = floatx4_s{0.0f, 0.0f, 0.0f, 0.0f};
+  const int steps = g.K / 64, s_end = steps * (wave + 1) / WAVES;
+  u32x4_s bf[8], af[2][MB];
+  auto fetch = [&](int s) {
+    const long k = static_cast<long>(s) * 64;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) red[((wave * (MB * 4) + m * 4 + n) * 4 + v) * 64 + lane] = acc[m][n][v];
-  __syncthreads();
-  bool bad = false;
-  for (int blk = wave; blk < MB * 4; blk += WAVES) {
-    const int row = row0 + blk / 4 * 16 + l16, col = col0 + blk % 4 * 16 + kg * 4;
-    float x[4];
+    for (int i = 0; i < 8; ++i) bf[i] = *reinterpret_cast<const u32x4_s*>(b[i] + k);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      float part[WAVES];
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w) part[w] = red[((w * (MB * 4) + blk) * 4 + v) * 64 + lane];
+      for (int m = 0; m < MB; ++m) af[t][m] = *reinterpret_cast<const u32x4_s*>(a[m] + k + t * 32);
+  };
+  int s0 = steps * wave / WAVES;
+  if (s0 < s_end) fetch(s0);
+  for (; s0 < s_end; ++s0) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    u32x4_s am[2][MB];
 #pragma unroll
-      for (int span = 1; span < WAVES; span *= 2)
+    for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_s*>(own + (i * 8 + ncol) * KM_PITCH + piece * 16) = bf[i];
 #pragma unroll
-        for (int w = 0; w < WAVES; w += 2 * span) part[w] += part[w + span];
-      x[v] = part[0];
-    }
-    if (row < g.M && col < g.N)
-      bad |= PLAIN ? gemm_store4(g, 0, row, col, x[0], x[1], x[2], x[3]) : gemm_store4_epi(g, 0, row, col, x[0], x[1], x[2], x[3]);
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) am[t][m] = af[t][m];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (s0 + 1 < s_end) fetch(s0 + 1);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const u32x4_s w = *reinterpret_cast<const u32x4_s*>(own + (n * 16 + l16) * KM_PITCH + t * 64 + kg * 16);
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_s, w), __builtin_bit_cast(bf16x8_s, am[t][m]), acc[m][n], 0, 0, 0);
+      }
   }
-  if (bad) dev_raise_fault(g.fault, g.tag);
+  __syncthreads();
+  skinny_meet<MB, WAVES, PLAIN>(g, acc, reinterpret_cast<float*>(km_smem), row0, col0, wave, lane);
 }
 
 struct SkinnyTile {
@@ -321,15 +390,16 @@ int32_t launch_rows4(omx_ctx* ctx, const GemmArgs& g) {
   return OMX_OK;
 }
 
-template <int MB>
+template <int MB, bool B_KM>
 int32_t launch_km(omx_ctx* ctx, const GemmArgs& g) {
-  constexpr int WAVES = 8, smem = km_lds<MB, WAVES>();
-  auto kernel = g.epi == OMX_EPI_NONE ? &gemm_skinny_km_kernel<MB, WAVES, true> : &gemm_skinny_km_kernel<MB, WAVES, false>;
+  constexpr int WAVES = 8, smem = B_KM ? km_lds<MB, WAVES>() : kc_lds<MB, WAVES>();
+  auto kernel = B_KM ? (g.epi == OMX_EPI_NONE ? &gemm_skinny64_km_kernel<MB, WAVES, true> : &gemm_skinny64_km_kernel<MB, WAVES, false>)
+                     : (g.epi == OMX_EPI_NONE ? &gemm_skinny64_kc_kernel<MB, WAVES, true> : &gemm_skinny64_kc_kernel<MB, WAVES, false>);
   if constexpr (smem > 64 * 1024)
     OMX_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
   dim3 grid(static_cast<unsigned>((g.N + 63) / 64), static_cast<unsigned>((g.M + 16 * MB - 1) / (16 * MB)), static_cast<unsigned>(g.batches));
   omx_launch_timed(ctx, kernel, grid, dim3(WAVES * 64), smem, ctx->timing_start, ctx->timing_stop, g);
-  OMX_LAUNCH_CHECK(ctx, "gemm_skinny_km_kernel");
+  OMX_LAUNCH_CHECK(ctx, "gemm_skinny64_km_kernel");
   return OMX_OK;
 }
 
@@ -353,16 +423,18 @@ int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g) {
   }
 }
 
-// Row blocks of 16 that a workgroup of gemm_skinny_km_kernel takes, and what the product takes there, in us; negative: not one for it. One
+// Row blocks of 16 that a workgroup of the 64-column kernels takes, and what the product takes there, in us; negative: not one for them. One
 // block where that makes at most a workgroup per compute unit, else two where they do; a second round of workgroups is what
-// the 64 x 64 tiles gain by (400 x 2048 over 768: 7.0 there, 8.4 to 10 here). us of a call, 64 x 64 tiles / this kernel: 282 x 640 and 768
-// over 768 6.3 / 4.7, over 1280 7.9 / 6.0, over 2048 10.3 / 7.5; 64 x 1024 over 768 6.1 / 4.8; 400 x 1024 over 1280 8.4 / 7.1 (two
-// blocks); over 4096 columns of K and more the tiles' split reductions are ahead. Sums of eight short chains: errors the same or smaller.
-double omx_gemm_skinny_km_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int* mb) {
-  if (a_km || !b_km || g.K % 32 != 0 || g.K > 4096 || g.N % 8 != 0 || !g.a_vec || !g.b_vec || ctx->gemm_skinny_km == 0) return -1.0;
+// the 64 x 64 tiles gain by (400 x 2048 over 768: 7.0 there, 8.4 to 10 here). us of a call. B by rows of K, 64 x 64 tiles / here:
+// 282 x 640 and 768 over 768 6.3 / 4.7, over 1280 7.9 / 6.0, over 2048 10.3 / 7.5; 64 x 1024 over 768 6.1 / 4.8; 400 x 1024 over
+// 1280 8.4 / 7.1 (two blocks); over 4096 and more the tiles' split reductions are ahead. B's columns by K, gemm_skinny_kernel's
+// tiles of 16 x 32 and more / here: 200 x 640 over 2048 10.0 / 7.1, over 4096 17.1 / 10.9; 96 x 2048 over 3072 13.7 / 9.1; 512 x
+// 384 over 2048 10.1 / 7.2; its 16 x 16 tiles stay ahead (64 x 768 over 1280 5.1 / 5.9). Sums of eight short chains, as there.
+double omx_gemm_skinny64_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, int* mb) {
+  if (a_km || g.K % (b_km ? 32 : 64) != 0 || g.K > 4096 || (b_km && g.N % 8 != 0) || !g.a_vec || !g.b_vec || ctx->gemm_skinny64 == 0) return -1.0;
   const long units = ctx->cu_count > 0 ? ctx->cu_count : 256, cols = (g.N + 63l) / 64 * g.batches;
-  if (ctx->gemm_skinny_km > 0) {  // forced (a grid's rows of workgroups are 16 bits)
-    *mb = ctx->gemm_skinny_km;
+  if (ctx->gemm_skinny64 > 0) {  // forced (a grid's rows of workgroups are 16 bits)
+    *mb = ctx->gemm_skinny64;
     return g.M <= 1 << 16 ? 0.0 : -1.0;
   }
   *mb = (g.M + 15l) / 16 * cols <= units ? 1 : 2;
@@ -370,6 +442,7 @@ double omx_gemm_skinny_km_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_
   return *mb == 1 ? 2.6 + 2.2e-3 * g.K : 2.9 + 3.1e-3 * g.K;
 }
 
-int32_t omx_gemm_skinny_km_launch(omx_ctx* ctx, const GemmArgs& g, int mb) {
-  return mb == 1 ? launch_km<1>(ctx, g) : launch_km<2>(ctx, g);
+int32_t omx_gemm_skinny64_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km, int mb) {
+  if (!b_km) return mb == 1 ? launch_km<1, false>(ctx, g) : launch_km<2, false>(ctx, g);
+  return mb == 1 ? launch_km<1, true>(ctx, g) : launch_km<2, true>(ctx, g);
 }

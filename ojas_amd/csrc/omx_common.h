@@ -139,7 +139,7 @@ struct omx_ctx {
   int adamw_trust = 1;        // 0: omx_adamw_step_bounded always runs its checking pass
   int ce_fused = 1;           // 0: linear-CE always takes the separate statistics and gradient kernels
   int sdpa_tiled = 1;         // 0: f32 attention always takes the one-wave-per-row kernels
-  int gemm_skinny_km = -1;    // few rows by a k-major B: -1: by rule; 0: never; 1, 2: wherever it fits, that many 16-row blocks a workgroup
+  int gemm_skinny64 = -1;    // few rows on 64 columns a workgroup: -1: by rule; 0: never; 1, 2: wherever it fits, that many 16-row blocks a workgroup
   int muon_symmetric = 1;     // 0: bf16 Newton-Schulz forms both halves of X X^T and b A + c A^2
   int muon_fused_sums = 1;    // 0: Newton-Schulz forms b A + c A^2 and a X + B X in kernels of their own
   bool profile_gemm = false;

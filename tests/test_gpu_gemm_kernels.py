@@ -915,8 +915,9 @@ def test_weight_gradients_of_a_few_heads(be, m, k, n, lda, count, bf16_out):
 
 @pytest.mark.parametrize("blocks", [1, 2])
 @pytest.mark.parametrize("m,k,n,count", [(1, 32, 8, 1), (15, 64, 64, 1), (17, 288, 72, 2), (33, 1280, 200, 1), (64, 736, 640, 1), (282, 544, 136, 1), (100, 4096, 64, 3)])
-def test_few_rows_by_rows_of_k(be, m, k, n, count, blocks):
-    """`gemm_skinny_km_kernel`, an input gradient of few rows: f32 and bf16 outputs, accumulation, ragged rows and columns, waves without a
+@pytest.mark.parametrize("by_k", [False, True])
+def test_few_rows_on_64_columns_a_workgroup(be, m, k, n, count, blocks, by_k):
+    """`gemm_skinny64_km_kernel` and `_kc_kernel`, linear layers and their input gradients of few rows: f32 and bf16 outputs, accumulation, ragged rows and columns, waves without a
     step. f32 sums of exact products: within k roundings of the terms' size."""
     from ojas_amd.backend import BF16, F32
 
@@ -926,18 +927,21 @@ def test_few_rows_by_rows_of_k(be, m, k, n, count, blocks):
     ar, br = be.download_f32(da).astype(np.float64), be.download_f32(db).astype(np.float64)
     want, size = ar @ br, np.abs(ar) @ np.abs(br)
     bound = size * k * 2.0**-24
+    strides = (1, k) if by_k else (n, 1)
+    if by_k:
+        db = be.upload(np.ascontiguousarray(b.transpose(0, 2, 1)), BF16)
     try:
-        be.set_option("gemm_skinny_km", blocks)
+        be.set_option("gemm_skinny64", blocks)
         for dtype in (F32, BF16):
             if count == 1:
-                got = be.gemm(da, (k, 1), db, (n, 1), m, k, n, dtype)
+                got = be.gemm(da, (k, 1), db, strides, m, k, n, dtype)
             else:
-                got = be.gemm_strided_batch(da, (k, 1), db, (n, 1), m, k, n, count, (m * k, k * n, m * n), dtype)
+                got = be.gemm_strided_batch(da, (k, 1), db, strides, m, k, n, count, (m * k, k * n, m * n), dtype)
             got = be.download_f32(got).reshape(want.shape)
             assert np.all(np.abs(got - want) <= bound + (np.abs(want) * 2.0**-8 if dtype == BF16 else 0))
         if count == 1:
             start = rng.normal(0, 1, (m, n)).astype(np.float32)
-            got = be.download(be.gemm(da, (k, 1), db, (n, 1), m, k, n, F32, be.upload(start)))
+            got = be.download(be.gemm(da, (k, 1), db, strides, m, k, n, F32, be.upload(start)))
             assert np.all(np.abs(got - (want[0] + start)) <= bound[0] + (np.abs(want[0]) + np.abs(start)) * 2.0**-23)
     finally:
-        be.set_option("gemm_skinny_km", -1)
+        be.set_option("gemm_skinny64", -1)
