@@ -405,12 +405,13 @@ int32_t launch_km(omx_ctx* ctx, const GemmArgs& g) {
 
 }  // namespace
 
-// What the product takes here, in us (see skinny_tile); negative: not one for this kernel. An activation's store pass over
-// sixteen blocks takes 2.5 us more (2048 x 512 over K = 512: 9.3 us, 5.5 on 64 x 64 tiles).
+// What the product takes here, in us (see skinny_tile); negative: not one for this kernel. Sixteen blocks' sums meet in 1.7 us more, and go
+// through an activation in 2.6 (2048 x 512 over K = 512: 9.3 us, 5.5 on 64 x 64 tiles; 700 to 2048 rows by 384 and 512 columns over
+// 128 / 256 / 384 5.2 / 6.2 / 7.4, which those take 4.0 / 4.5 / 4.9 for).
 double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, bool activation) {
   if (a_km || b_km || g.K % 32 != 0 || !g.a_vec || !g.b_vec) return -1.0;
   const int t = skinny_tile(g, ctx->cu_count > 0 ? ctx->cu_count : 256);
-  return t < 0 ? -1.0 : 2.5 + 1e-3 * g.K * (SKINNY_TILES[t].mb + SKINNY_TILES[t].nb) + (activation && t == 3 ? 2.5 : 0.0);
+  return t < 0 ? -1.0 : 2.5 + 1e-3 * g.K * (SKINNY_TILES[t].mb + SKINNY_TILES[t].nb) + (t == 3 ? (activation ? 2.6 : 1.7) : 0.0);
 }
 
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g) {
