@@ -681,7 +681,8 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   const double skinny_us = operand_dtype == OMX_BF16 && !thin && !low_rank && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
                                ? omx_gemm_skinny_us(ctx, g, a_km, b_km, epi && epi->mode != OMX_EPI_NONE) : -1.0;
   int blocks64 = 0;
-  const double us64 = operand_dtype == OMX_BF16 && !thin && !low_rank && !heads && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
+  // (With a low-rank term from 1024 columns of K on: below, a widened int8 weight's product keeps the one chain, and the bits, of the codes'.)
+  const double us64 = operand_dtype == OMX_BF16 && !thin && !heads && (!low_rank || k >= 1024) && ctx->gemm_dma_mode == 1 && ctx->gemm_forced_tiling < 0
                            ? omx_gemm_skinny64_us(ctx, g, a_km, b_km, &blocks64) : -1.0;
   bool skinny64 = us64 >= 0.0 && (skinny_us < 0.0 || us64 < skinny_us), skinny = skinny_us >= 0.0 && !heads && !skinny64;
   int frag32 = -1, dma32 = -1;
@@ -948,7 +949,7 @@ int32_t omx_gemm_impl(omx_ctx* ctx, uint32_t fault_op, const void* a, uint64_t a
   }
   g.lr_rank = g.lr_block_cols = 0;
   if (low_rank) {
-    if (dma_variant < 0) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: no kernel for a low-rank term at this shape", op);
+    if (dma_variant < 0 && !skinny64) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: no kernel for a low-rank term at this shape", op);
     g.lr_h = static_cast<const unsigned short*>(low_rank->h);
     g.lr_w = static_cast<const unsigned short*>(low_rank->w);
     g.lr_pitch = static_cast<long>(low_rank->h_pitch);

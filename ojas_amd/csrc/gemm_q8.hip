@@ -500,7 +500,7 @@ int32_t set_low_rank(omx_ctx* ctx, const char* op, Q8Args* g, const omx_low_rank
 // the codes. gemm_q8_kernel's widening rides on four of eight waves and holds it at 950 TFLOP/s, one tiling whatever the shape;
 // the bf16 kernels do 1070 to 1360 on the same products and have small tiles for small ones. The weight's values are the same; the
 // sums over K are one chain in the same order, and the same bits, unless omx_gemm_impl shares K between launches (few tiles,
-// K >= 2048) or waves (few rows or columns, no low-rank term): f32 sums in another order, no further from the f64 product. (In one
+// K >= 2048) or waves (few rows or columns; with a low-rank term K >= 1024): f32 sums in another order, no further from the f64 product. (In one
 // chain at any shape, few rows would lose what the copy gives them: 64 rows over 8192 -> 2048 123 us over the codes, 23 over the
 // copy, 44 so.) Estimates in us: a 32-column step of gemm_q8_kernel 0.46 alone on a compute unit, 1.06 with two there; the copy 3.5
 // and 3.1 bytes a weight at 4.5 TB/s. us over codes and over the copy, forward / input gradient: 8192 rows over 2048 x 16384: 590,

@@ -155,6 +155,32 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows4_kernel(GemmArgs g) {
   }
 }
 
+// The low-rank term of a workgroup's rows and columns, by one wave: operands straight from memory, 32 of the rank a step (16 past its end are
+// zeros).
+template <int MB>
+__device__ __forceinline__ void skinny_low_rank(const GemmArgs& g, floatx4_s (&acc)[MB][4], int row0, int col0, int lane) {
+  const int l16 = lane & 15, kg = lane >> 4;
+#pragma unroll 1
+  for (int p = kg * 8; p - kg * 8 < g.lr_rank; p += 32) {
+    u32x4_s w[4], h[4][MB];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const long off = g.lr_block_cols > 0 ? static_cast<long>(min(col0 + n * 16, g.N - 1) / g.lr_block_cols) * g.lr_rank : 0;
+      w[n] = u32x4_s{0u, 0u, 0u, 0u};
+      if (p < g.lr_rank) w[n] = *reinterpret_cast<const u32x4_s*>(g.lr_w + min(col0 + n * 16 + l16, g.N - 1) * g.lr_w_pitch + p);
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        h[n][m] = u32x4_s{0u, 0u, 0u, 0u};
+        if (p < g.lr_rank) h[n][m] = *reinterpret_cast<const u32x4_s*>(g.lr_h + min(row0 + m * 16 + l16, g.M - 1) * g.lr_pitch + off + p);
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_s, w[n]), __builtin_bit_cast(bf16x8_s, h[n][m]), acc[m][n], 0, 0, 0);
+  }
+}
 // The waves' sums over 16 MB rows x 64 columns meet and go out: acc[m][n][v] is row m * 16 + lane % 16, column n * 16 + 4 * (lane / 16) + v.
 template <int MB, int WAVES, bool PLAIN>
 __device__ __forceinline__ void skinny_meet(const GemmArgs& g, const floatx4_s (&acc)[MB][4], float* red, int row0, int col0, int wave, int lane) {
@@ -262,6 +288,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny64_km_kernel(GemmArgs g
         }
       }
   }
+  if (g.lr_rank > 0 && wave == 0) skinny_low_rank<MB>(g, acc, row0, col0, lane);  // (no wave has fewer steps)
   __syncthreads();  // the steps' LDS has been read
   skinny_meet<MB, WAVES, PLAIN>(g, acc, reinterpret_cast<float*>(km_smem), row0, col0, wave, lane);
 }
@@ -327,6 +354,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny64_kc_kernel(GemmArgs g
           acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_s, w), __builtin_bit_cast(bf16x8_s, am[t][m]), acc[m][n], 0, 0, 0);
       }
   }
+  if (g.lr_rank > 0 && wave == 0) skinny_low_rank<MB>(g, acc, row0, col0, lane);
   __syncthreads();
   skinny_meet<MB, WAVES, PLAIN>(g, acc, reinterpret_cast<float*>(km_smem), row0, col0, wave, lane);
 }
@@ -440,7 +468,7 @@ double omx_gemm_skinny64_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_k
   }
   *mb = (g.M + 15l) / 16 * cols <= units ? 1 : 2;
   if (*mb == 2 && (g.M + 31l) / 32 * cols > units) return -1.0;
-  return *mb == 1 ? 2.6 + 2.2e-3 * g.K : 2.9 + 3.1e-3 * g.K;
+  return *mb == 1 ? 2.6 + 2.2e-3 * g.K : b_km ? 2.9 + 3.1e-3 * g.K : 3.2 + 3.3e-3 * g.K;
 }
 
 int32_t omx_gemm_skinny64_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km, int mb) {

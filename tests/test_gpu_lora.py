@@ -453,3 +453,37 @@ def test_lora_adapter_starts_as_the_identity(be):
         assert tr.loss_and_grads() == loss0
     finally:
         tr.close()
+
+
+@pytest.mark.parametrize("rows,k,cols,rank,block", [(40, 1024, 192, 16, 0), (213, 1152, 384, 32, 128), (17, 2048, 64, 48, 0), (300, 1088, 136 * 8, 16, 0)])
+@pytest.mark.parametrize("backward", [False, True])
+def test_low_rank_term_of_few_rows_over_a_long_reduction(be, rows, k, cols, rank, block, backward):
+    """The 64-column kernels of few rows with the low-rank term beside the waves' shares of K: within k + rank roundings of the f64 product's
+    terms (exact products of bf16 values, f32 sums), and a bf16 output's own."""
+    from ojas_amd.backend import BF16
+
+    print(f"q8 low-rank few rows={rows} k={k} cols={cols} rank={rank} backward={backward}", flush=True)
+    block = 0 if backward else block
+    rng = np.random.default_rng(rows + k)
+    nout, kin = (k, cols) if backward else (cols, k)
+    codes, scales = rng.integers(-127, 128, (nout, kin)).astype(np.int8), np.full((nout, kin // 32), 2.0**-8, np.float32)
+    bf = lambda a: orc.round_bf16(a.astype(np.float32))
+    x, w = bf(rng.normal(0, 1, (rows, k))), bf(rng.normal(0, 0.3, (cols, rank)))
+    blocks = cols // block if block else 1
+    h = bf(rng.normal(0, 1, (rows, blocks * rank)))
+    low_rank = (be.upload(h, BF16), be.upload(w, BF16), block)
+    weight = bf(codes.astype(np.float32) * 2.0**-8).astype(np.float64)
+    weight = weight if backward else weight.T
+    want, size = x.astype(np.float64) @ weight, np.abs(x).astype(np.float64) @ np.abs(weight)
+    for i in range(blocks):
+        at = slice(i * block, (i + 1) * block) if block else slice(None)
+        hi = h[:, i * rank:(i + 1) * rank].astype(np.float64)
+        want[:, at] += hi @ w[at].T
+        size[:, at] += np.abs(hi) @ np.abs(w[at]).T
+    be.set_option("q8_widen", 1)
+    try:
+        args = (be.upload(codes), be.upload(scales), be.upload(x, BF16))
+        y = be.linear_i8_group_backward_input(*args, low_rank=low_rank) if backward else be.linear_i8_group_forward(args[2], *args[:2], low_rank=low_rank)
+    finally:
+        be.set_option("q8_widen", -1)
+    assert np.all(np.abs(be.download_f32(y) - want) <= size * (k + rank) * 2.0**-24 + np.abs(want) * 2.0**-8)
