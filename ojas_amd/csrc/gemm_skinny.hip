@@ -433,13 +433,14 @@ int32_t launch_km(omx_ctx* ctx, const GemmArgs& g) {
 
 }  // namespace
 
-// What the product takes here, in us (see skinny_tile); negative: not one for this kernel. Sixteen blocks' sums meet in 1.7 us more, and go
-// through an activation in 2.6 (2048 x 512 over K = 512: 9.3 us, 5.5 on 64 x 64 tiles; 700 to 2048 rows by 384 and 512 columns over
-// 128 / 256 / 384 5.2 / 6.2 / 7.4, which those take 4.0 / 4.5 / 4.9 for).
+// What the product takes here, in us; negative: not one for this kernel. Kernel times by tile (46 shapes of 48 to 1024 rows over 128 to 768; the
+// last, whose sixteen blocks' sums meet, 700 to 2048 rows: 5.2 / 6.2 / 7.4 over 128 / 256 / 384, which 64 x 64 tiles take 4.0 / 4.5 /
+// 4.9 for; with an activation a microsecond more: 2048 x 512 over 512 9.3, 5.5 there).
 double omx_gemm_skinny_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_km, bool activation) {
   if (a_km || b_km || g.K % 32 != 0 || !g.a_vec || !g.b_vec) return -1.0;
   const int t = skinny_tile(g, ctx->cu_count > 0 ? ctx->cu_count : 256);
-  return t < 0 ? -1.0 : 2.5 + 1e-3 * g.K * (SKINNY_TILES[t].mb + SKINNY_TILES[t].nb) + (t == 3 ? (activation ? 2.6 : 1.7) : 0.0);
+  static constexpr double kBase[4] = {2.45, 2.85, 2.9, 4.2}, kColumn[4] = {1.9e-3, 2.7e-3, 3.8e-3, 8.1e-3};
+  return t < 0 ? -1.0 : kBase[t] + kColumn[t] * g.K + (activation && t == 3 ? 1.0 : 0.0);
 }
 
 int32_t omx_gemm_skinny_launch(omx_ctx* ctx, const GemmArgs& g) {
@@ -468,7 +469,10 @@ double omx_gemm_skinny64_us(omx_ctx* ctx, const GemmArgs& g, bool a_km, bool b_k
   }
   *mb = (g.M + 15l) / 16 * cols <= units ? 1 : 2;
   if (*mb == 2 && (g.M + 31l) / 32 * cols > units) return -1.0;
-  return *mb == 1 ? 2.6 + 2.2e-3 * g.K : b_km ? 2.9 + 3.1e-3 * g.K : 3.2 + 3.3e-3 * g.K;
+  // Kernel times. By rows of K a sixth less, for the 64 x 64 tiles take half a microsecond more there than their estimate says (512 x 256 over
+  // 128 4.0, here 3.4).
+  if (b_km) return 0.85 * (*mb == 1 ? 3.2 + 1.8e-3 * g.K : 3.4 + 2.5e-3 * g.K);
+  return *mb == 1 ? 3.35 + 1.85e-3 * g.K : 3.7 + 2.75e-3 * g.K;
 }
 
 int32_t omx_gemm_skinny64_launch(omx_ctx* ctx, const GemmArgs& g, bool b_km, int mb) {
