@@ -44,6 +44,7 @@ constexpr int flash_dkv_set(int D) { return 2 * 64 * D * 2 + 2 * 64 * 4; }  // b
 constexpr int FLASH_OWN_ROWS = 1024;                    // row terms that a key side's workgroup keeps for itself
 constexpr int flash_dq_lds(int D, int groups) { return groups * 4 * ftile(D) + D * 4; }
 constexpr int flash_dkv_waves(int D, int groups) { return D == 64 && groups <= 2 ? 2 : 1; }
+constexpr bool flash_in_turn(int D, int groups) { return D > 64 || groups > 1; }  // (see flash_fwd_tile)
 // Waves per SIMD the query-side passes are compiled for: what their LDS leaves room for.
 constexpr int flash_waves(int D, int groups) { return groups == 1 ? (D == 64 ? 3 : 2) : groups == 2 && D == 64 ? 2 : 1; }
 
@@ -309,15 +310,35 @@ __device__ __forceinline__ void flash_block_of(int pairs, int planes, int* pair,
   }
 }
 
+// use(i, load(i)) for i = 0 .. N - 1, a load two uses ahead of its own. Left to itself the compiler reads an operand out of LDS right
+// before the product that takes it (one set of registers, a full LDS latency a product), which few waves a SIMD do not hide.
+// Forward and dQ pass of head_dim 128, 13 x 9 heads x 1177 rows: 107 -> 99 and 146 -> 138 us; 8 x 3 x 531: 19.1 -> 16.9 and 21.0 ->
+// 19.1; one key tile, nothing else on the chip: 6.7 -> 6.5. Three and five ahead measure the same.
+template <int N, typename Load, typename Use>
+__device__ __forceinline__ void in_turn(Load&& load, Use&& use) {
+  constexpr int AHEAD = 2 < N ? 2 : N;
+  constexpr int VECTOR_SCALAR = 6;  // what may move across: vector and scalar arithmetic, neither reads nor products
+  u32x4 f[AHEAD + 1];
+  for_sequence<AHEAD>([&](auto i) { f[i.value] = load(i); });
+  for_sequence<N>([&](auto i) {
+    if constexpr (i.value + AHEAD < N) f[(i.value + AHEAD) % (AHEAD + 1)] = load(std::integral_constant<int, i.value + AHEAD>{});
+    __builtin_amdgcn_sched_barrier(VECTOR_SCALAR);
+    use(i, f[i.value % (AHEAD + 1)]);
+    __builtin_amdgcn_sched_barrier(VECTOR_SCALAR);
+  });
+}
+
 // ------------------------------------------------------------------ forward
 // One 32-query x 64-key tile of one wave: scores, online softmax, weights times values.
 //   NSUB      32-key halves of the tile that hold a visible key (the second half of a tile whose
 //             first key is the wave's first query is hidden from all 32 rows and is left out);
 //   MASK_SUB  the half the causal diagonal cuts (its keys start at the wave's first query), or -1;
 //   GENERAL   the tile crosses the sequence end or a window edge: every element is tested.
+//   IN_TURN   operands are read two products ahead (in_turn). Not at head_dim 64 with three waves a SIMD: the registers end (10
+//             spilled, 46.2 against 46.3 us at 16 x 12 x 1024 and 37.2 against 36.6 at 12 x 12 x 999), and the waves fill in.
 // `m` is the running maximum of the raw scores; the scale joins inside the fma. `lsum` sums the
 // weights as computed, `wsum` their bf16 copies (this lane's half of the keys).
-template <int D, int NSUB, int MASK_SUB, bool GENERAL>
+template <int D, int NSUB, int MASK_SUB, bool GENERAL, bool IN_TURN>
 __device__ __forceinline__ void flash_fwd_tile(const char* k_rows, const char* v_rows, const u32x4 (&qf)[D / 16],
                                                floatx16 (&o)[D / 32], float& m, float& lsum, float& wsum,
                                                float scale_log2, int key0, int q_row, int T, int window, int lane) {
@@ -329,11 +350,20 @@ __device__ __forceinline__ void flash_fwd_tile(const char* k_rows, const char* v
   // A wave in its vector phase therefore holds up the others' products for the whole phase; raised
   // priority for the two short product phases keeps the matrix units fed (7 % on the forward pass).
   __builtin_amdgcn_s_setprio(2);
+  if constexpr (IN_TURN) {
+    in_turn<NSUB * KK>([&](auto i) { return frag_rows<D>(k_rows, i.value / KK, i.value % KK, l32, lg); },
+                       [&](auto i, const u32x4& f) {
+                         constexpr int sub = i.value / KK, kk = i.value % KK;
+                         if constexpr (kk == 0) sc[sub] = zero16();
+                         sc[sub] = mfma(f, qf[kk], sc[sub]);
+                       });
+  } else {
 #pragma unroll
-  for (int sub = 0; sub < NSUB; ++sub) {
-    sc[sub] = zero16();
+    for (int sub = 0; sub < NSUB; ++sub) {
+      sc[sub] = zero16();
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) sc[sub] = mfma(frag_rows<D>(k_rows, sub, kk, l32, lg), qf[kk], sc[sub]);
+      for (int kk = 0; kk < KK; ++kk) sc[sub] = mfma(frag_rows<D>(k_rows, sub, kk, l32, lg), qf[kk], sc[sub]);
+    }
   }
   __builtin_amdgcn_s_setprio(0);
   if constexpr (GENERAL) {
@@ -406,15 +436,28 @@ __device__ __forceinline__ void flash_fwd_tile(const char* k_rows, const char* v
   lsum += psum;
   m = new_m;
   __builtin_amdgcn_s_setprio(2);
+  u32x4 pb;
+  auto weights = [&](auto sub, auto c) {
+    pb = pack8(sc[sub], c);
+    wsum = sum_pairs(pb.x, sum_pairs(pb.y, sum_pairs(pb.z, sum_pairs(pb.w, wsum))));
+  };
+  if constexpr (IN_TURN) {
+    in_turn<NSUB * 2 * MT>([&](auto i) { return frag_tr<D>(v_rows, i.value % MT, i.value / (2 * MT), i.value / MT % 2, lane); },
+                           [&](auto i, const u32x4& f) {
+                             constexpr int mt = i.value % MT;
+                             if constexpr (mt == 0) weights(i.value / (2 * MT), i.value / MT % 2);
+                             o[mt] = mfma(f, pb, o[mt]);
+                           });
+  } else {
 #pragma unroll
-  for (int sub = 0; sub < NSUB; ++sub)
+    for (int sub = 0; sub < NSUB; ++sub)
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const u32x4 pb = pack8(sc[sub], c);
-      wsum = sum_pairs(pb.x, sum_pairs(pb.y, sum_pairs(pb.z, sum_pairs(pb.w, wsum))));
+      for (int c = 0; c < 2; ++c) {
+        weights(sub, c);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) o[mt] = mfma(frag_tr<D>(v_rows, mt, sub, c, lane), pb, o[mt]);
-    }
+        for (int mt = 0; mt < MT; ++mt) o[mt] = mfma(frag_tr<D>(v_rows, mt, sub, c, lane), pb, o[mt]);
+      }
+  }
   __builtin_amdgcn_s_setprio(0);
 }
 
@@ -515,7 +558,7 @@ __global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_fwd_kernel(c
         advance(kt);
         const int key0 = kt * 64;
         if ((GROUPS == 1 || kt <= kt_last) && key0 <= wave_q0 + 31 && key0 + 63 + s.window > wave_q0)
-          flash_fwd_tile<D, 2, -1, true>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, s.window, lane);
+          flash_fwd_tile<D, 2, -1, true, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, s.window, lane);
       }
     } else if (wave_q0 < T) {  // (a wave whose rows all lie past the sequence end only keeps the barriers)
       // The wave's first query is a multiple of 32 and a tile's first key a multiple of 64, so the
@@ -526,17 +569,17 @@ __global__ __launch_bounds__(FT, flash_waves(D, GROUPS)) void flash_fwd_kernel(c
       const int diag_kt = wave_q0 / 64;
       for (; kt < diag_kt; kt += GROUPS) {
         advance(kt);
-        flash_fwd_tile<D, 2, -1, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, kt * 64, q_row, T, 0, lane);
+        flash_fwd_tile<D, 2, -1, false, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, kt * 64, q_row, T, 0, lane);
       }
       if (GROUPS == 1 || kt == diag_kt) {
         advance(kt);
         const int key0 = kt * 64;
         if (D > 64 || key0 + 63 >= T)  // (at head_dim 128 the two cut-tile forms cost registers the kernel does not have)
-          flash_fwd_tile<D, 2, -1, true>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
+          flash_fwd_tile<D, 2, -1, true, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
         else if (key0 == wave_q0)
-          flash_fwd_tile<D, 1, 0, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
+          flash_fwd_tile<D, 1, 0, false, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
         else
-          flash_fwd_tile<D, 2, 1, false>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
+          flash_fwd_tile<D, 2, 1, false, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, o, m, lsum, wsum, scale_log2, key0, q_row, T, 0, lane);
         kt += GROUPS;
       }
     }
@@ -1130,11 +1173,11 @@ __device__ __forceinline__ void flash_dq_tile(const char* k_rows, const char* v_
 #pragma unroll
   for (int sub = 0; sub < 2; ++sub) {
     floatx16 sc = zero16(), dp = zero16();
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      sc = mfma(frag_rows<D>(k_rows, sub, kk, l32, lg), qf[kk], sc);
-      dp = mfma(frag_rows<D>(v_rows, sub, kk, l32, lg), gf[kk], dp);
-    }
+    in_turn<2 * KK>([&](auto i) { return frag_rows<D>(i.value % 2 ? v_rows : k_rows, sub, i.value / 2, l32, lg); },
+                                    [&](auto i, const u32x4& f) {
+                                      if constexpr (i.value % 2 == 0) sc = mfma(f, qf[i.value / 2], sc);
+                                      else dp = mfma(f, gf[i.value / 2], dp);
+                                    });
     if constexpr (GENERAL) {
 #pragma unroll
       for (int vv = 0; vv < 16; ++vv) {
@@ -1148,13 +1191,15 @@ __device__ __forceinline__ void flash_dq_tile(const char* k_rows, const char* v_
       const float p = __builtin_amdgcn_exp2f(fmaf(sc[vv], scale_log2, neg_lse));
       dp[vv] = p * (dp[vv] - row_del);  // dS / scale: the scale joins dQ at the end
     }
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const u32x4 dsb = pack8(dp, c);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) dq[mt] = mfma(frag_tr<D>(k_rows, mt, sub, c, lane), dsb, dq[mt]);
-      ds_sum = sum_pairs(dsb.x, sum_pairs(dsb.y, sum_pairs(dsb.z, sum_pairs(dsb.w, ds_sum))));
-    }
+    u32x4 dsb;
+    in_turn<2 * MT>([&](auto i) { return frag_tr<D>(k_rows, i.value % MT, sub, i.value / MT, lane); },
+                                    [&](auto i, const u32x4& f) {
+                                      if constexpr (i.value % MT == 0) {
+                                        dsb = pack8(dp, i.value / MT);
+                                        ds_sum = sum_pairs(dsb.x, sum_pairs(dsb.y, sum_pairs(dsb.z, sum_pairs(dsb.w, ds_sum))));
+                                      }
+                                      dq[i.value % MT] = mfma(f, dsb, dq[i.value % MT]);
+                                    });
   }
 }
 
