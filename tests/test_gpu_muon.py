@@ -460,3 +460,33 @@ def test_half_formed_symmetric_products_carry_the_whole_ones_bits(be, rows, cols
     for a, b in zip(got[1], got[0]):
         assert np.array_equal(a, b)
     assert any(np.any(a != p) for a, p in zip(got[1][:count], ps))
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(1, 3), (3, 5), (33, 50), (64, 48), (97, 97), (515, 1030)])
+def test_tensors_off_16_bytes_carry_the_aligned_ones_bits(be, rows, cols, bf16):
+    """The passes around the iteration take four elements a lane where the tensors lie on 16 bytes, else one, and the last elements of a
+    count that is no multiple of four by themselves: the same bits, and nothing behind the tensors."""
+    from ojas_amd.backend import BF16, F32, DeviceTensor, MuonNs5Config
+
+    print(f"muon off 16 bytes {rows}x{cols} bf16 {bf16}", flush=True)
+    r = np.random.default_rng(rows + 3 * cols)
+    n = rows * cols
+    p, g, m = (r.standard_normal(n).astype(np.float32) * k for k in (0.1, 0.03, 0.01))
+    got = []
+    for lead in (0, 1, 2):
+        def at(x, dtype):
+            whole = be.upload(np.concatenate([np.full(lead, 7.0, np.float32), x, np.full(9, 7.0, np.float32)]), dtype)
+            return whole, DeviceTensor(be, whole.ptr + lead * (2 if dtype == BF16 else 4), (rows, cols), dtype, owns=False)
+
+        held = [at(p, F32), at(g, F32), at(m, F32), at(np.zeros(n, np.float32), BF16)]
+        tensors = [t for _, t in held]
+        be.muon_ns5_step_batched([tensors[0]], [tensors[1]], [tensors[2]], MuonNs5Config(0.02, 0.95, 0.1, 1, bf16), [tensors[3]])
+        be.sync()
+        parts = [be.download_f32(whole) for whole, _ in held]
+        assert all(np.all(x[:lead] == 7.0) and np.all(x[lead + n:] == 7.0) for x in parts)
+        got.append([x[lead:lead + n] for x in parts])
+    assert not np.array_equal(got[0][0], p)
+    assert np.array_equal(got[0][1], g)
+    for other in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(got[0], other))
