@@ -437,6 +437,13 @@ int32_t omx_adamw_step_bounded(omx_ctx* ctx, void* param_f32, const void* grad_f
                                void* moment1_f32, void* moment2_f32, uint64_t n, uint64_t step,
                                const omx_adamw_config* config, void* param_bf16,
                                int32_t inputs_bounded, void* unbounded_flag);
+/* omx_adamw_step_bounded on the gradient times `grad_scale` (0 .. 1, omx_clip_scale's), which is written back: the bits of
+ * omx_clip_grad_norm and the step after it in one pass less over the gradient. It is scaled also where the step is refused, though not where
+ * an argument is null, n is 0 or the scale is none. */
+int32_t omx_adamw_step_scaled(omx_ctx* ctx, void* param_f32, void* grad_f32,
+                              void* moment1_f32, void* moment2_f32, uint64_t n, uint64_t step,
+                              const omx_adamw_config* config, void* param_bf16,
+                              int32_t inputs_bounded, void* unbounded_flag, float grad_scale);
 /* omx_adamw_step on `count` tensors in one set of launches (a small model's tens of vectors), bit for bit what
  * a call for each gives, in the list's order where tensors overlap: each tensor is all-or-nothing by itself. The arrays
  * hold device pointers. */
@@ -480,6 +487,9 @@ uint64_t omx_muon_scratch_bytes(uint64_t rows, uint64_t cols);
  * coefficient (clip_scale, backend.rs:277-303) is below 1 (a tensor that is listed twice, twice). A sync point. */
 int32_t omx_clip_grad_norm(omx_ctx* ctx, void* const* grads_f32, const uint64_t* lens,
                            uint64_t count, float max_norm, float* norm_out);
+/* omx_clip_grad_norm without the scaling: the factor, at most 1, is the caller's to apply. A sync point. */
+int32_t omx_clip_scale(omx_ctx* ctx, const void* const* grads_f32, const uint64_t* lens,
+                       uint64_t count, float max_norm, float* norm_out, float* scale_out);
 
 /* ---- elementwise and layout ---- */
 /* BackendFloat::residual_add_forward (backend.rs:1165-1173): out = x + y, one

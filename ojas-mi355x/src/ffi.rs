@@ -120,6 +120,7 @@ extern "C" {
     pub fn omx_embedding_backward_accumulate(ctx: *mut OmxCtx, ids_u32: *const c_void, grad: *const c_void, grad_dtype: i32, table_grad_f32: *mut c_void, tokens: u64, vocab: u64, dim: u64) -> i32;
     pub fn omx_adamw_step(ctx: *mut OmxCtx, param_f32: *mut c_void, grad_f32: *const c_void, moment1_f32: *mut c_void, moment2_f32: *mut c_void, n: u64, step: u64, config: *const OmxAdamwConfig, param_bf16: *mut c_void) -> i32;
     pub fn omx_adamw_step_bounded(ctx: *mut OmxCtx, param_f32: *mut c_void, grad_f32: *const c_void, moment1_f32: *mut c_void, moment2_f32: *mut c_void, n: u64, step: u64, config: *const OmxAdamwConfig, param_bf16: *mut c_void, inputs_bounded: i32, unbounded_flag: *mut c_void) -> i32;
+    pub fn omx_adamw_step_scaled(ctx: *mut OmxCtx, param_f32: *mut c_void, grad_f32: *mut c_void, moment1_f32: *mut c_void, moment2_f32: *mut c_void, n: u64, step: u64, config: *const OmxAdamwConfig, param_bf16: *mut c_void, inputs_bounded: i32, unbounded_flag: *mut c_void, grad_scale: f32) -> i32;
     pub fn omx_adamw_step_batched(ctx: *mut OmxCtx, params_f32: *const *mut c_void, grads_f32: *const *const c_void, moments1_f32: *const *mut c_void, moments2_f32: *const *mut c_void, lens: *const u64, count: u64, step: u64, config: *const OmxAdamwConfig) -> i32;
     pub fn omx_muon_ns5_step(ctx: *mut OmxCtx, param_f32: *mut c_void, grad_f32: *const c_void, momentum_f32: *mut c_void, rows: u64, cols: u64, config: *const OmxMuonConfig, param_bf16: *mut c_void) -> i32;
     pub fn omx_muon_ns5_step_batched(ctx: *mut OmxCtx, params_f32: *const *mut c_void, grads_f32: *const *const c_void, momenta_f32: *const *mut c_void, params_bf16: *const *mut c_void, count: u64, rows: u64, cols: u64, config: *const OmxMuonConfig) -> i32;
@@ -127,6 +128,7 @@ extern "C" {
     pub fn omx_muon_ns5_step_shapes(ctx: *mut OmxCtx, params_f32: *const *mut c_void, grads_f32: *const *const c_void, momenta_f32: *const *mut c_void, params_bf16: *const *mut c_void, rows: *const u64, cols: *const u64, count: u64, config: *const OmxMuonConfig) -> i32;
     pub fn omx_muon_scratch_bytes(rows: u64, cols: u64) -> u64;
     pub fn omx_clip_grad_norm(ctx: *mut OmxCtx, grads_f32: *const *mut c_void, lens: *const u64, count: u64, max_norm: f32, norm_out: *mut f32) -> i32;
+    pub fn omx_clip_scale(ctx: *mut OmxCtx, grads_f32: *const *const c_void, lens: *const u64, count: u64, max_norm: f32, norm_out: *mut f32, scale_out: *mut f32) -> i32;
     pub fn omx_residual_add(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, y: *const c_void, y_dtype: i32, out: *mut c_void, out_dtype: i32, n: u64) -> i32;
     pub fn omx_accumulate_grad(ctx: *mut OmxCtx, acc_f32: *mut c_void, grad_f32: *const c_void, n: u64) -> i32;
     pub fn omx_accumulate_grads(ctx: *mut OmxCtx, accs_f32: *const *mut c_void, grads_f32: *const *const c_void, lens: *const u64, count: u64) -> i32;

@@ -599,16 +599,16 @@ int32_t ogpt_step(ogpt* t, const omx_adamw_config* adamw, float grad_clip, float
   if (!t || !adamw) return OMX_BACKEND;
   TRY(gradients(t));
   // Sync point 1: the global gradient norm is a host value (trainer.rs:821-824).
-  void* grads[1] = {t->g32};
+  const void* grads[1] = {t->g32};
   uint64_t lens[1] = {t->P};
-  float norm = 0.0f;
-  TRY(omx_clip_grad_norm(t->ctx, grads, lens, 1, grad_clip > 0.0f ? grad_clip : INFINITY, &norm));
-  // One AdamW pass over the arena covers every tensor; the bf16 mirror is refreshed in the same pass.
+  float norm = 0.0f, scale = 1.0f;
+  TRY(omx_clip_scale(t->ctx, grads, lens, 1, grad_clip > 0.0f ? grad_clip : INFINITY, &norm, &scale));
+  // One AdamW pass over the arena covers every tensor; the gradients are clipped and the bf16 mirror refreshed in the same pass.
   int32_t bounded = 0;
   TRY(adamw_inputs_bounded(t, ogpt::kFull, norm, &bounded));
   t->tracked = ogpt::kNone;  // until the readback below has seen this step through
-  TRY(omx_adamw_step_bounded(t->ctx, t->p32, t->g32, t->m1, t->m2, t->P, t->steps, adamw, t->p16, bounded,
-                             t->unbounded));
+  TRY(omx_adamw_step_scaled(t->ctx, t->p32, t->g32, t->m1, t->m2, t->P, t->steps, adamw, t->p16, bounded,
+                             t->unbounded, scale));
   // Sync point 2: sync + the step's one readback.
   float l = 0.0f;
   TRY(read_loss_and_flag(t, &l));

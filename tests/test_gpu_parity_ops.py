@@ -756,6 +756,48 @@ def test_adamw_bounded_form_skips_the_check_only_when_nothing_can_overflow(be):
     assert got[4] is not None and got[4].code == NON_FINITE and np.array_equal(got[0], p)
 
 
+@pytest.mark.parametrize("n,lead", [(1, 0), (3, 0), (4, 0), (4, 1), (1027, 0), (1027, 2), (300_001, 0)])
+@pytest.mark.parametrize("mirror", [False, True])
+def test_adamw_on_a_scaled_gradient_is_clip_and_step_in_turn(be, n, lead, mirror):
+    """`omx_clip_scale` and `omx_adamw_step_scaled`: every bit of `omx_clip_grad_norm` and `omx_adamw_step_bounded` after it, the gradient
+    included, in one pass (unchecked, 16-byte aligned) or two; a refused step finds its gradient scaled all the same."""
+    import ctypes as C
+
+    from ojas_amd.backend import BF16, F32, NON_FINITE, AdamWConfig, DeviceTensor, OjasError
+
+    print(f"adamw scaled {n} at {lead}", flush=True)
+    r = np.random.default_rng(n + lead)
+    p, g, m1 = (r.standard_normal(n).astype(np.float32) for _ in range(3))
+    m2 = np.square(r.standard_normal(n)).astype(np.float32)
+    config = AdamWConfig.nanolab(1e-2, 0.1)
+    limit = C.c_float(0.25 * float(np.linalg.norm(g)))
+
+    def run(fused, bounded, spoil):
+        wholes = [be.upload(np.concatenate([np.full(lead, 7.0, np.float32), x, np.full(5, 7.0, np.float32)])) for x in (np.full(n, spoil, np.float32) if spoil else p, g, m1, m2)]
+        dp, dg, d1, d2 = (DeviceTensor(be, w.ptr + 4 * lead, (n,), F32, owns=False) for w in wholes)
+        bf16 = be.upload(np.zeros(n, np.float32), BF16) if mirror else None
+        flag = be.upload(np.zeros(1, np.uint32))
+        ptrs, lens = (C.c_void_p * 1)(dg.ptr), (C.c_uint64 * 1)(n)
+        norm, scale = C.c_float(), C.c_float(1.0)
+        tail = [C.c_uint64(n), C.c_uint64(3), C.byref(config), be._p(bf16) if mirror else None, C.c_int32(bounded), be._p(flag)]
+        if fused:
+            be._check(be._lib.omx_clip_scale(be._ctx, ptrs, lens, C.c_uint64(1), limit, C.byref(norm), C.byref(scale)))
+            assert 0.2 < scale.value < 0.3
+            be._check(be._lib.omx_adamw_step_scaled(be._ctx, be._p(dp), be._p(dg), be._p(d1), be._p(d2), *tail, scale))
+        else:
+            be._check(be._lib.omx_clip_grad_norm(be._ctx, ptrs, lens, C.c_uint64(1), limit, C.byref(norm)))
+            be._check(be._lib.omx_adamw_step_bounded(be._ctx, be._p(dp), be._p(dg), be._p(d1), be._p(d2), *tail))
+        if spoil:
+            with pytest.raises(OjasError) as e:
+                be.sync()
+            assert e.value.code == NON_FINITE
+        return [np.float32(norm.value)] + [be.download(x) for x in wholes + [flag] + ([bf16] if mirror else [])]
+
+    for bounded, spoil in ((1, 0.0), (0, 0.0), (0, np.inf)):
+        for a, b in zip(run(True, bounded, spoil), run(False, bounded, spoil)):
+            assert np.array_equal(a, b)
+
+
 def test_adamw_config_refusals(be):
     from ojas_amd.backend import NON_FINITE, OUT_OF_RANGE, AdamWConfig, OjasError
 
