@@ -611,6 +611,14 @@ int32_t omx_linear_swiglu_forward(omx_ctx* ctx, const void* x, const void* w, in
 int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32,
                                            uint64_t group, int32_t layout, void* gate_up, void* out, uint64_t rows, uint64_t kin,
                                            uint64_t hidden);
+/* A weight of int8 codes meets its activations twice in a training step, and a product over a widened copy of it (see "q8_widen") can leave
+ * that copy for the other: the next int8 product keeps it `offset` bytes (a multiple of 256) into a scratch of `total` bytes (8 GiB at most).
+ * `formed`: 0, or what omx_i8_copy_formed said after an earlier product over the same codes at the same offset and total, whose copy is then
+ * read as it is unless the scratch was given back since: any allocation that would be refused takes it back, and no copy is kept in the
+ * context from then on. The caller sees to it that nothing else was kept there in between and that the codes are what they were.
+ * omx_i8_copy_formed: 0 where the last int8 product kept no copy. */
+int32_t omx_i8_copy_next(omx_ctx* ctx, uint64_t offset, uint64_t total, uint64_t formed);
+uint64_t omx_i8_copy_formed(const omx_ctx* ctx);
 /* The input gradient of linear_backward (backend.rs:1628-1645) of the projection behind a SwiGLU, w [out, hidden] bf16, and swiglu_backward of
  * it: every bit of g_gate_up [rows, 2 hidden] bf16 as those two calls have it. scratch [rows, hidden] bf16 holds the product where it takes
  * two launches; what it holds afterwards is not defined. The second form over int8 codes (omx_linear_i8_group_backward_input, gate_up f32). */

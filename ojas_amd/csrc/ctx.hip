@@ -219,17 +219,17 @@ bool capturing(const omx_ctx* ctx) {
   return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 
-// Whether drop_extra gives workspace `slot` (kExtraSlot or kSumsSlot) back: not while the op that runs uses it, a graph holds its
+// Whether drop_extra gives workspace `slot` (one that ops can do without) back: not while the op that runs uses it, a graph holds its
 // address or a capture is on.
 bool droppable(const omx_ctx* ctx, int slot) {
-  return ctx->workspace[slot] && !(slot == kExtraSlot && ctx->extra_in_use) && !ctx->workspace_captured[slot] && !capturing(ctx);
+  return ctx->workspace[slot] && slot != ctx->slot_in_use && !ctx->workspace_captured[slot] && !capturing(ctx);
 }
 
-// Gives workspaces kExtraSlot and kSumsSlot back, with the sums that wait there formed. Whether there was one. (No op allocates
+// Gives workspaces kExtraSlot, kSumsSlot and kCopiesSlot back, with the sums that wait there formed. Whether there was one. (No op allocates
 // between omx_partial_rows and its omx_column_sum.)
 bool drop_extra(omx_ctx* ctx) {
   bool dropped = false;
-  for (int slot : {kExtraSlot, kSumsSlot}) {
+  for (int slot : {kExtraSlot, kSumsSlot, kCopiesSlot}) {
     void*& held = ctx->workspace[slot];
     if (!droppable(ctx, slot) || (slot == kSumsSlot && omx_form_sums(ctx) != OMX_OK)) continue;
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return dropped;
@@ -238,6 +238,7 @@ bool drop_extra(omx_ctx* ctx) {
     (void)hipFree(held);
     held = nullptr;
     ctx->workspace_bytes[slot] = 0;
+    ctx->copies_dropped |= slot == kCopiesSlot;
     dropped = true;
   }
   return dropped;
@@ -481,8 +482,8 @@ bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot) {
   if (bytes <= held || ctx->budget_limit == 0) return true;
   uint64_t back = ctx->workspace_captured[slot] || capturing(ctx) ? 0 : held;  // what growing it gives back
   // An op's plan does not depend on what others can do without: omx_alloc takes that back for it.
-  if (slot != kExtraSlot && slot != kSumsSlot)
-    for (int extra : {kExtraSlot, kSumsSlot})
+  if (!can_do_without(slot))
+    for (int extra : {kExtraSlot, kSumsSlot, kCopiesSlot})
       if (droppable(ctx, extra)) back += ctx->workspace_bytes[extra];
   return ctx->budget_live - back + workspace_size(bytes) <= ctx->budget_limit;
 }
@@ -517,6 +518,7 @@ int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot) {
   if (rc != OMX_OK) return rc;
   ctx->workspace_bytes[slot] = rounded;
   ctx->workspace_captured[slot] = in_graph;
+  if (slot == kCopiesSlot) ++ctx->copies_generation;
   *out = ctx->workspace[slot];
   return OMX_OK;
 }

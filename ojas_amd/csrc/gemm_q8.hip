@@ -20,6 +20,7 @@
 // HBM traffic per product: the activation once per column band, the codes once per row band at
 // ONE byte per weight, the scales at one eighth of that.
 #include <algorithm>
+#include <utility>
 
 #include "gemm_tiles.h"
 
@@ -506,40 +507,70 @@ int32_t set_low_rank(omx_ctx* ctx, const char* op, Q8Args* g, const omx_low_rank
 // and 3.1 bytes a weight at 4.5 TB/s. us over codes and over the copy, forward / input gradient: 8192 rows over 2048 x 16384: 590,
 // 525 / 552, 421; over 2048 x 2048: 77, 70 / 76, 65; 1024 rows there: 34, 26 / 37, 27; 64 rows over 2048 x 6144: 35, 25 / 100, 25.
 // The other way round, and left: 8192 rows over 512 -> 4096: 49, 58; 512 over 2048 -> 16384: 48, 64.
-bool widen_pays(const omx_ctx* ctx, uint64_t m, uint64_t k, uint64_t n) {
+// `share`: how much of the copy is this product's to pay.
+bool widen_pays(const omx_ctx* ctx, uint64_t m, uint64_t k, uint64_t n, double share) {
   if (ctx->q8_widen >= 0) return ctx->q8_widen != 0;
   const double cus = ctx->cu_count > 0 ? ctx->cu_count : 256, tiles = static_cast<double>((m + QBM - 1) / QBM * ((n + QBN - 1) / QBN));
   const double over_codes = 4.0 + static_cast<double>(k / QBK) * (tiles <= cus ? 0.46 : 1.06 * std::max(1.0, tiles / (2.0 * cus)));
-  const double over_copy = 3.5 + static_cast<double>(k) * static_cast<double>(n) * 6.9e-7 + omx_gemm_bf16_us(ctx, m, k, n);
+  const double over_copy = share * (3.5 + static_cast<double>(k) * static_cast<double>(n) * 6.9e-7) + omx_gemm_bf16_us(ctx, m, k, n);
   return over_copy < 0.93 * over_codes;
 }
 int32_t widened_product(omx_ctx* ctx, uint32_t fault_op, const Q8Args& g, uint64_t rows, uint64_t kin, uint64_t nout,
-                        bool backward, bool* taken, const OmxGemmEpilogue* epi = nullptr) {
+                        bool backward, bool* taken, const OmxI8Copy& keep, const OmxGemmEpilogue* epi = nullptr) {
   *taken = false;
   const uint64_t k = backward ? nout : kin, n = backward ? kin : nout;
-  constexpr uint64_t kMost = 1ull << 30;  // bytes of scratch
-  if (g.add || nout * kin * 2 > kMost || !widen_pays(ctx, rows, k, n) || !omx_gemm_takes_low_rank(ctx, g.a, k, nullptr, kin, k)) return OMX_OK;
-  unsigned short* w = static_cast<unsigned short*>(omx_workspace_if_room(ctx, nout * kin * 2, kExtraSlot));
-  if (!w) return OMX_OK;
-  const long pieces = static_cast<long>(nout) * static_cast<long>(kin / 8);
-  omx_launch(ctx, q8_widen_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, g.codes, g.scales, w,
-             static_cast<long>(nout), static_cast<long>(kin), g.packed);
-  OMX_LAUNCH_CHECK(ctx, "q8_widen_kernel");
+  constexpr uint64_t kMost = 1ull << 30, kMostKept = 8ull << 30;  // bytes of scratch
+  const uint64_t bytes = nout * kin * 2;
+  // A copy that is kept for a later product over the same codes (omx_i8_copy_next): half of it is that one's to pay.
+  bool kept = keep.total > 0 && keep.total <= kMostKept && keep.offset <= keep.total && bytes <= keep.total - keep.offset && keep.offset % 256 == 0 && !ctx->copies_dropped;
+  const bool there = kept && keep.formed != 0 && keep.formed == ctx->copies_generation && ctx->workspace[kCopiesSlot] && ctx->workspace_bytes[kCopiesSlot] >= keep.total;
+  if (g.add || bytes > kMost || !widen_pays(ctx, rows, k, n, there ? 0.0 : kept && !backward ? 0.5 : 1.0) || !omx_gemm_takes_low_rank(ctx, g.a, k, nullptr, kin, k)) {
+    if (there) ctx->copy_formed = keep.formed;
+    return OMX_OK;
+  }
+  char* at = kept ? static_cast<char*>(omx_workspace_if_room(ctx, keep.total, kCopiesSlot)) : nullptr;
+  if (at) {
+    at += keep.offset;
+  } else if (kept) {
+    kept = false;
+    ctx->copies_dropped = true;  // (not to be asked for again at every product)
+  }
+  if (!kept) at = static_cast<char*>(omx_workspace_if_room(ctx, bytes, kExtraSlot));
+  if (!at) return OMX_OK;
+  unsigned short* w = reinterpret_cast<unsigned short*>(at);
+  if (kept) ctx->copy_formed = ctx->copies_generation;
+  if (!(kept && there)) {
+    const long pieces = static_cast<long>(nout) * static_cast<long>(kin / 8);
+    omx_launch(ctx, q8_widen_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, g.codes, g.scales, w,
+               static_cast<long>(nout), static_cast<long>(kin), g.packed);
+    OMX_LAUNCH_CHECK(ctx, "q8_widen_kernel");
+  }
   const OmxLowRank lr{g.lr_h, g.lr_w, static_cast<uint64_t>(g.lr_pitch), static_cast<uint64_t>(g.lr_w_pitch),
                       static_cast<uint64_t>(g.lr_rank), static_cast<uint64_t>(g.lr_block_cols)};
-  ctx->extra_in_use = true;
+  ctx->slot_in_use = kept ? kCopiesSlot : kExtraSlot;
   const int32_t rc = omx_gemm_impl(ctx, fault_op, g.a, k, 1, w, backward ? kin : 1, backward ? 1 : kin, OMX_BF16, g.c,
                                    g.c_f32 ? OMX_F32 : OMX_BF16, n, rows, k, n, 0, epi, nullptr, 0, g.lr_rank > 0 ? &lr : nullptr);
-  ctx->extra_in_use = false;
+  ctx->slot_in_use = -1;
   // Partial sums that there is no room for: the codes' kernel has none.
   *taken = rc != OMX_CAPACITY_EXCEEDED;
   return *taken ? rc : OMX_OK;
+}
+
+// What omx_i8_copy_next asked of this product. (Every int8 product takes it, a refused one too.)
+OmxI8Copy take_copy(omx_ctx* ctx) {
+  ctx->copy_formed = 0;
+  return std::exchange(ctx->copy_next, {});
+}
+int32_t refuse_null(omx_ctx* ctx, const char* op) {
+  take_copy(ctx);
+  return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
 }
 
 // `after`: OMX_EPI_SWIGLU or OMX_EPI_ROPE of the product.
 int32_t i8_forward(omx_ctx* ctx, const char* op, const void* x, int32_t x_dtype, const void* codes_i8, const void* scales_f32, uint64_t group,
                    int32_t layout, const void* add, const omx_low_rank* low_rank, void* y, int32_t y_dtype, uint64_t rows, uint64_t kin,
                    uint64_t nout, const OmxGemmEpilogue* after) {
+  const OmxI8Copy keep = take_copy(ctx);
   int32_t rc = check_q8(ctx, op, x, codes_i8, scales_f32, y, add, rows, kin, nout, group, x_dtype, layout);
   if (rc != OMX_OK) return rc;
   if (!omx_valid_float_dtype(y_dtype)) return omx_fail(ctx, OMX_DTYPE, "%s: the output must be f32 or bf16", op);
@@ -564,7 +595,7 @@ int32_t i8_forward(omx_ctx* ctx, const char* op, const void* x, int32_t x_dtype,
   rc = set_low_rank(ctx, op, &g, low_rank, nout);
   if (rc != OMX_OK) return rc;
   bool taken = false;
-  rc = widened_product(ctx, F_LINEAR_FORWARD, g, rows, kin, nout, false, &taken, after);
+  rc = widened_product(ctx, F_LINEAR_FORWARD, g, rows, kin, nout, false, &taken, keep, after);
   if (rc != OMX_OK || taken) return rc;
   g.tag = omx_tag(ctx, F_LINEAR_FORWARD);
   rc = launch_q8<false>(ctx, g, 2.0 * rows * kin * nout);
@@ -580,6 +611,7 @@ int32_t i8_forward(omx_ctx* ctx, const char* op, const void* x, int32_t x_dtype,
 int32_t i8_backward_input(omx_ctx* ctx, const char* op, const void* codes_i8, const void* scales_f32, uint64_t group, int32_t layout, const void* gy,
                           int32_t gy_dtype, const void* add, const omx_low_rank* low_rank, void* gx, uint64_t rows, uint64_t kin, uint64_t nout,
                           const OmxGemmEpilogue* after) {
+  const OmxI8Copy keep = take_copy(ctx);
   int32_t rc = check_q8(ctx, op, gy, codes_i8, scales_f32, gx, add, rows, kin, nout, group, gy_dtype, layout);
   if (rc != OMX_OK) return rc;
   if (nout % 32 != 0)
@@ -603,7 +635,7 @@ int32_t i8_backward_input(omx_ctx* ctx, const char* op, const void* codes_i8, co
   rc = set_low_rank(ctx, op, &g, low_rank, kin);
   if (rc != OMX_OK) return rc;
   bool taken = false;
-  rc = widened_product(ctx, F_LINEAR_BACKWARD, g, rows, kin, nout, true, &taken, after);
+  rc = widened_product(ctx, F_LINEAR_BACKWARD, g, rows, kin, nout, true, &taken, keep, after);
   if (rc != OMX_OK || taken) return rc;
   g.tag = omx_tag(ctx, F_LINEAR_BACKWARD);
   rc = launch_q8<true>(ctx, g, 2.0 * rows * kin * nout);
@@ -613,6 +645,14 @@ int32_t i8_backward_input(omx_ctx* ctx, const char* op, const void* codes_i8, co
 }  // namespace
 
 extern "C" {
+
+int32_t omx_i8_copy_next(omx_ctx* ctx, uint64_t offset, uint64_t total, uint64_t formed) {
+  OMX_REQUIRE_CTX(ctx);
+  ctx->copy_next = {offset, total, formed};
+  return OMX_OK;
+}
+
+uint64_t omx_i8_copy_formed(const omx_ctx* ctx) { return ctx ? ctx->copy_formed : 0; }
 
 int32_t omx_linear_i8_group_forward(omx_ctx* ctx, const void* x, int32_t x_dtype, const void* codes_i8,
                                     const void* scales_f32, uint64_t group, int32_t layout, const void* add,
@@ -626,7 +666,7 @@ int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t 
                                            int32_t layout, void* gate_up, void* out, uint64_t rows, uint64_t kin, uint64_t hidden) {
   OMX_REQUIRE_CTX(ctx);
   const char* op = "linear_i8_group_swiglu_forward";
-  if (!out) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (!out) return refuse_null(ctx, op);
   const OmxGemmEpilogue pairs = {OMX_EPI_SWIGLU, 0, nullptr, out};
   return i8_forward(ctx, op, x, x_dtype, codes_i8, scales_f32, group, layout, nullptr, nullptr, gate_up, OMX_F32, rows, kin, 2 * hidden, &pairs);
 }
@@ -637,7 +677,7 @@ int32_t omx_linear_i8_group_rope_forward(omx_ctx* ctx, const void* x, int32_t x_
                                          uint64_t dim) {
   OMX_REQUIRE_CTX(ctx);
   const char* op = "linear_i8_group_rope_forward";
-  if (!out || !cos_f32 || !sin_f32) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (!out || !cos_f32 || !sin_f32) return refuse_null(ctx, op);
   if (time == 0 || dim == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
   if (time > 0x7fffffffull || dim > 0x7fffffffull || heads > 0x7fffffffull || plain_heads > 0x7fffffffull || (heads + plain_heads) * dim > 0x7fffffffull)
     return omx_fail(ctx, OMX_OUT_OF_RANGE, "%s: axis does not fit in i32", op);
@@ -662,7 +702,7 @@ int32_t omx_linear_i8_group_backward_input_swiglu(omx_ctx* ctx, const void* code
                                                   uint64_t rows, uint64_t hidden, uint64_t nout) {
   OMX_REQUIRE_CTX(ctx);
   const char* op = "linear_i8_group_backward_input_swiglu";
-  if (!gate_up || !g_gate_up) return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+  if (!gate_up || !g_gate_up) return refuse_null(ctx, op);
   const OmxGemmEpilogue pairs = {OMX_EPI_SWIGLU_BWD, 0, gate_up, g_gate_up};
   return i8_backward_input(ctx, op, codes_i8, scales_f32, group, layout, gy, gy_dtype, nullptr, nullptr, scratch, rows, hidden, nout, &pairs);
 }
@@ -672,7 +712,7 @@ int32_t omx_pack_i8_group(omx_ctx* ctx, const void* codes_i8, const void* scales
   OMX_REQUIRE_CTX(ctx);
   const char* op = "pack_i8_group";
   if (!codes_i8 || !scales_f32 || !blocked_codes || !blocked_scales)
-    return omx_fail(ctx, OMX_PLACEMENT, "%s: null device pointer", op);
+    return refuse_null(ctx, op);
   if (group != 32) return omx_fail(ctx, OMX_UNSUPPORTED, "%s: group size %llu (only 32)", op, (unsigned long long)group);
   if (nout == 0 || kin == 0) return omx_fail(ctx, OMX_SHAPE, "%s: zero-sized axis", op);
   if (kin % 128 != 0 || nout % 8 != 0)

@@ -84,6 +84,9 @@ struct OmxParked {
   uint64_t last = 0, before = 0;
 };
 
+struct OmxI8Copy {
+  uint64_t offset = 0, total = 0, formed = 0;
+};
 struct omx_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -109,15 +112,19 @@ struct omx_ctx {
   // Slot 0: per-op scratch. Slot 1: split-K partials of the GEMM (which an op
   // may call while it holds slot 0) and operands converted for an op that holds slot 0.
   // Slot 2: tensors an op keeps across calls into other ops (a recomputed attention output).
-  void* workspace[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
-  uint64_t workspace_bytes[5] = {0, 0, 0, 0, 0};
-  bool extra_in_use = false;  // workspace kExtraSlot, by the op that runs
+  void* workspace[6] = {};
+  uint64_t workspace_bytes[6] = {};
+  int slot_in_use = -1;  // kExtraSlot or kCopiesSlot, by the op that runs
+  // The copy that the next int8 product keeps (omx_i8_copy_next), and what its copy, or the last one's, is known by.
+  OmxI8Copy copy_next;
+  uint64_t copy_formed = 0, copies_generation = 0;  // (the second: blocks that were workspace kCopiesSlot so far)
+  bool copies_dropped = false;                      // an allocation needed their memory: no more of them
   // Column sums that wait (omx_defer_weight_sums), their partial rows in workspace kSumsSlot up to sums_used.
   bool sums_wait = false, prepare_sums_wait = false;
   uint32_t sums_expected = 0;
   uint64_t sums_used = 0;
   std::vector<OmxColumnSum> sums;
-  bool workspace_captured[5] = {false, false, false, false, false};  // handed out while the stream was captured
+  bool workspace_captured[6] = {};  // handed out while the stream was captured
   int cu_count = 0;
   // This device's copy of the static scratch of omx_cross_entropy_mean_forward_static, looked up
   // when the context is opened (the lookup is not stream work and may load the code object).
@@ -219,11 +226,13 @@ struct OmxKernelTimer {
 };
 
 int32_t omx_hip_fail(omx_ctx* ctx, hipError_t err, const char* what);
-// Workspaces kExtraSlot and kSumsSlot are for what an op can do without: any allocation that would be refused takes them back first.
-constexpr int kExtraSlot = 3, kSumsSlot = 4;
+// Workspaces kExtraSlot, kSumsSlot and kCopiesSlot are for what an op can do without: any allocation that would be refused takes them back
+// first.
+constexpr int kExtraSlot = 3, kSumsSlot = 4, kCopiesSlot = 5;
+constexpr bool can_do_without(int slot) { return slot >= kExtraSlot; }
 // Grows workspace `slot` to at least `bytes` (budget-charged).
 int32_t omx_workspace(omx_ctx* ctx, uint64_t bytes, void** out, int slot = 0);
-// Whether the budget has room for workspace `slot` at that size (for an op that can do with less), counting what kExtraSlot and kSumsSlot
+// Whether the budget has room for workspace `slot` at that size (for an op that can do with less), counting what those three
 // would give back.
 bool omx_workspace_fits(const omx_ctx* ctx, uint64_t bytes, int slot = 0);
 // Workspace `slot` for an op that can do without: null where the budget or the device lacks the room, and where a capture would have to

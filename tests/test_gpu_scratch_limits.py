@@ -502,3 +502,60 @@ def test_norm_backward_of_few_rows_asks_for_the_scratch_that_it_uses(waits):
         want = orc.rms_norm_backward(x, w, gy)
         close(gx, want[0])
         close(gw, want[1])
+
+
+@pytest.mark.parametrize("rows,kin,nout,rank", [(5, 256, 512, 0), (67, 1408, 1024, 16), (130, 1024, 1408, 0), (1042, 1280, 896, 16)])
+def test_a_kept_copy_of_a_weight_gives_the_bits_of_a_copy_of_its_own(rows, kin, nout, rank):
+    """`omx_i8_copy_next`: forward products leave their widened copies for the input gradients. The same bits as copies formed for each, with
+    two weights in the scratch, after an allocation took it back (no copy is kept from then on), and with a mark that another block gave."""
+    import ctypes as C
+
+    from ojas_amd.backend import BF16, F32, MiBackend
+
+    print(f"kept copies {rows} x {kin} -> {nout}, rank {rank}", flush=True)
+    r = np.random.default_rng(rows + nout)
+    weights = [(r.integers(-127, 128, (nout, kin)).astype(np.int8), r.uniform(1e-4, 1e-3, (nout, kin // 32)).astype(np.float32)) for _ in range(2)]
+    xs, gs = (r.normal(0, 1, (rows, n)).astype(np.float32) for n in (kin, nout))
+    size = (2 * nout * kin + 255) // 256 * 256
+    budget = 96 << 20
+    be = MiBackend(0, budget_bytes=budget)
+    try:
+        be.set_option("q8_widen", 1)
+        ws = [tuple(be.upload(t) for t in w) for w in weights]
+        x, g = be.upload(xs, BF16), be.upload(gs, BF16)
+        tails = [None, None]
+        if rank:
+            tails = [tuple(be.upload(r.normal(0, 0.1, (n, rank)).astype(np.float32), BF16) for n in (rows, cols)) + (0,) for cols in (nout, kin)]
+
+        def both(copies, formed=None):
+            ys, left = [], []
+            for i, w in enumerate(ws):
+                if copies:
+                    be._check(be._lib.omx_i8_copy_next(be._ctx, C.c_uint64(i * size), C.c_uint64(2 * size), C.c_uint64(0)))
+                ys.append(be.linear_i8_group_forward(x, *w, low_rank=tails[0]))
+                left.append(formed or be._lib.omx_i8_copy_formed(be._ctx))
+            yield left
+            for i, w in enumerate(ws):
+                if copies:
+                    be._check(be._lib.omx_i8_copy_next(be._ctx, C.c_uint64(i * size), C.c_uint64(2 * size), C.c_uint64(left[i])))
+                ys.append(be.linear_i8_group_backward_input(*w, g, low_rank=tails[1]))
+            yield [be.download_f32(y) for y in ys]
+
+        be._lib.omx_i8_copy_formed.restype = C.c_uint64
+        left, want = both(False)
+        assert left == [0, 0]
+        left, got = both(True)
+        assert left[0] != 0 and left[0] == left[1]
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        _, got = both(True, formed=left[0] + 7)  # not this block's: formed anew
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        pair = both(True)
+        assert next(pair)[0] == left[0]
+        rest = be.empty(((budget - be.budget()["live"] + (1 << 20)) // 4,), F32)
+        del rest  # (a MiB more than there was: the scratch went back)
+        assert all(np.array_equal(a, b) for a, b in zip(next(pair), want))
+        left, got = both(True)
+        assert left == [0, 0]
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    finally:
+        be.close()
