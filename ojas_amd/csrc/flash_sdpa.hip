@@ -1440,13 +1440,19 @@ FlashShape make_shape(uint64_t batch, uint64_t heads, uint64_t kv_heads, uint64_
 // pairs fill the places exactly the lighter blocks still help: a compute unit serves its oldest
 // workgroup first, so equal workgroups that start together end one after another (30, 38 and 45 us
 // measured for the three of a unit), and the light blocks of the second half fill that tail
-// (forward 43.2 -> 42.1 us at 768 pairs). `also_rounds`: also when the pairs need more than one
-// round, whose last would run part empty (the blocks go out heaviest first).
-int flash_single(omx_ctx* ctx, unsigned pair_groups, int per_cu, bool also_rounds) {
+// (forward 43.2 -> 42.1 us at 768 pairs). Over a few rounds of places pairs end with a round that runs part empty, where single blocks
+// go out heaviest first: up to `rounds` of them. Beyond, a plane's blocks, which single ones spread over the whole grid, find its
+// tiles in an L2 no longer. us of pairs and of single blocks, forward / dQ, by how often the pairs fill the places: head_dim 128, 96 planes
+// x 1500 (1.12) 117, 93 / 157, 139; 117 x 1177 (1.14) 98, 80 / 125, 110; 256 x 700 (1.5) 72, 71 / 96, 102; 200 x 900 (1.56) 92, 85 / 137,
+// 121; 144 x 1500 (1.69) 125, 119 / 186, 167; 117 x 2048 (1.83) 181, 187 / 256, 254; 256 x 900 (2) 97, 113 / 146, 153; head_dim 64, 200 x
+// 900 (1.04) 58, 45 / 78, 65; 384 x 531 (1.5) 43, 38 / 63, 54; 512 x 700 (2) 70, 69 / 106, 108; 200 x 2048 (2.08) 167, 152 / 229, 218; 256 x
+// 2048 (2.67) 199, 215 / 311, 300.
+// dK/dV (two places a unit) of pairs and of single blocks: head_dim 128, 200 x 2048 (3.1) 590, 599; 256 x 2048 (4) 738, 765; 512 x 1177
+// (5) 624, 668; under four blocks, whose pairs are uneven, 1024 x 260 228, 195; head_dim 64 the same everywhere (512 x 1500 437, 435), and
+// 100, 86 at 1024 x 260.
+int flash_single(omx_ctx* ctx, unsigned pair_groups, int per_cu, double rounds) {
   if (ctx->flash_schedule != 0) return ctx->flash_schedule == 2 ? 0 : 1;  // forced (tests cover both)
-  const unsigned places = static_cast<unsigned>(ctx->cu_count > 0 ? ctx->cu_count : 256) * per_cu;
-  if (pair_groups <= places) return 1;
-  return also_rounds ? 1 : 0;
+  return pair_groups <= (ctx->cu_count > 0 ? ctx->cu_count : 256) * per_cu * rounds ? 1 : 0;
 }
 
 // f(integral_constant) of a group count the kernels of head dim D are compiled for.
@@ -1499,7 +1505,7 @@ void launch_forward(omx_ctx* ctx, const unsigned short* q, const unsigned short*
   // chance (two groups / one: 0.81 to 1.28). At 2048 columns it is 0.99 on average from 768 positions on, but 1.03 to 1.10 on each of four
   // models over 512, so there, where groups gain 0.4 to 4 us (16 heads x 128 / 512: 8.4 -> 8.0, 18.8 -> 14.6), one group stays.
   const int groups = D == 128 && tiles < 12 && ctx->flash_schedule == 0 ? 1 : flash_groups(ctx, planes, s.time, tiles, s.window > 0, D);
-  s.q_single = groups > 1 || flash_single(ctx, (q_blocks + 1) / 2 * planes, D == 64 ? 3 : 2, false);
+  s.q_single = groups > 1 || flash_single(ctx, (q_blocks + 1) / 2 * planes, D == 64 ? 3 : 2, D == 64 ? 2.25 : 1.75);
   const unsigned rows = 128 / groups;
   dim3 grid((s.q_single ? (s.time + rows - 1) / rows : (q_blocks + 1) / 2) * planes), block(FT);
   // Causal-counted work: half of the 4 B H T^2 D of the two full products.
@@ -1677,8 +1683,8 @@ void launch_backward(omx_ctx* ctx, const unsigned short* q, const unsigned short
   s.kv_parts = parts ? plan.parts : 1;
   const int kv_groups = s.kv_parts > 1 ? plan.groups : plan.whole_groups;
   const unsigned q_rows = 128 / q_groups, kv_rows = 128 / kv_groups;
-  s.q_single = q_groups > 1 || flash_single(ctx, pairs * q_planes, D == 64 ? 3 : 2, false);
-  s.kv_single = kv_groups > 1 || flash_single(ctx, pairs * kv_planes, 2, true);
+  s.q_single = q_groups > 1 || flash_single(ctx, pairs * q_planes, D == 64 ? 3 : 2, 1.75);
+  s.kv_single = kv_groups > 1 || flash_single(ctx, pairs * kv_planes, 2, D == 64 || s.time <= 384 ? 1e9 : 3.5);
   if (s.kv_parts > 1) s.kv_single = 1;
   dim3 kv_grid((s.kv_single ? (s.time + kv_rows - 1) / kv_rows : pairs) * kv_planes * s.kv_parts);
   dim3 q_grid((s.q_single ? (s.time + q_rows - 1) / q_rows : pairs) * q_planes);
