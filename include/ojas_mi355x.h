@@ -619,6 +619,11 @@ int32_t omx_linear_i8_group_swiglu_forward(omx_ctx* ctx, const void* x, int32_t 
  * omx_i8_copy_formed: 0 where the last int8 product kept no copy. */
 int32_t omx_i8_copy_next(omx_ctx* ctx, uint64_t offset, uint64_t total, uint64_t formed);
 uint64_t omx_i8_copy_formed(const omx_ctx* ctx);
+/* The copies of up to 8 weights, each where products over `rows` rows would run over one, in one launch: formed[i] as omx_i8_copy_formed says
+ * it for omx_i8_copy_next at offsets[i] of `total`, 0 where none was formed. Weights as omx_linear_i8_group_forward takes them. */
+int32_t omx_i8_copies_form(omx_ctx* ctx, const void* const* codes_i8, const void* const* scales_f32, const uint64_t* nout, const uint64_t* kin,
+                           const uint64_t* offsets, uint64_t count, uint64_t total, uint64_t group, int32_t layout, uint64_t rows,
+                           uint64_t* formed);
 /* The input gradient of linear_backward (backend.rs:1628-1645) of the projection behind a SwiGLU, w [out, hidden] bf16, and swiglu_backward of
  * it: every bit of g_gate_up [rows, 2 hidden] bf16 as those two calls have it. scratch [rows, hidden] bf16 holds the product where it takes
  * two launches; what it holds afterwards is not defined. The second form over int8 codes (omx_linear_i8_group_backward_input, gate_up f32). */

@@ -155,6 +155,7 @@ extern "C" {
     pub fn omx_linear_i8_group_swiglu_forward(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, codes_i8: *const c_void, scales_f32: *const c_void, group: u64, layout: i32, gate_up: *mut c_void, out: *mut c_void, rows: u64, kin: u64, hidden: u64) -> i32;
     pub fn omx_i8_copy_next(ctx: *mut OmxCtx, offset: u64, total: u64, formed: u64) -> i32;
     pub fn omx_i8_copy_formed(ctx: *const OmxCtx) -> u64;
+    pub fn omx_i8_copies_form(ctx: *mut OmxCtx, codes_i8: *const *const c_void, scales_f32: *const *const c_void, nout: *const u64, kin: *const u64, offsets: *const u64, count: u64, total: u64, group: u64, layout: i32, rows: u64, formed: *mut u64) -> i32;
     pub fn omx_linear_backward_input_swiglu(ctx: *mut OmxCtx, w: *const c_void, gy: *const c_void, operand_dtype: i32, gate_up: *const c_void, gate_up_dtype: i32, scratch: *mut c_void, g_gate_up: *mut c_void, rows: u64, hidden: u64, out_features: u64) -> i32;
     pub fn omx_linear_i8_group_backward_input_swiglu(ctx: *mut OmxCtx, codes_i8: *const c_void, scales_f32: *const c_void, group: u64, layout: i32, gy: *const c_void, gy_dtype: i32, gate_up: *const c_void, scratch: *mut c_void, g_gate_up: *mut c_void, rows: u64, hidden: u64, nout: u64) -> i32;
     pub fn omx_linear_i8_group_rope_forward(ctx: *mut OmxCtx, x: *const c_void, x_dtype: i32, codes_i8: *const c_void, scales_f32: *const c_void, group: u64, layout: i32, low_rank: *const OmxLowRank, scratch_f32: *mut c_void, out: *mut c_void, cos_f32: *const c_void, sin_f32: *const c_void, rows: u64, kin: u64, time: u64, heads: u64, plain_heads: u64, dim: u64) -> i32;

@@ -152,6 +152,25 @@ int32_t copy_left(olora* t, QMat& w, int32_t rc) {
   w.formed = omx_i8_copy_formed(t->ctx);
   return rc;
 }
+// A layer's copies in one launch where they are small (q8_widen_list_kernel): beyond, the launches fill the chip one by one and the first
+// product would find its copy further from it (67 million codes a layer, left to each product).
+constexpr uint64_t FEW_CODES = 32ull << 20;
+int32_t copies_of_layer(olora* t, olora::Layer& A) {
+  QMat* const all[4] = {&A.qkv, &A.o, &A.gu, &A.dn};
+  const void *codes[4], *scales[4];
+  uint64_t nout[4], kin[4], offsets[4], formed[4] = {0, 0, 0, 0}, sum = 0;
+  for (int i = 0; i < 4; ++i) {
+    codes[i] = all[i]->codes;
+    scales[i] = all[i]->scales;
+    nout[i] = all[i]->nout;
+    kin[i] = all[i]->kin;
+    offsets[i] = all[i]->copy_at;
+    sum += nout[i] * kin[i];
+  }
+  if (sum <= FEW_CODES) TRY(omx_i8_copies_form(t->ctx, codes, scales, nout, kin, offsets, 4, t->copies, 32, OMX_I8_BLOCKED, t->N, formed));
+  for (int i = 0; i < 4; ++i) all[i]->formed = formed[i];
+  return OMX_OK;
+}
 int32_t q8_forward(olora* t, const void* x, QMat& w, const omx_low_rank* lr, void* y_f32) {
   TRY(copy_of(t, w));
   return copy_left(t, w, omx_linear_i8_group_forward(t->ctx, x, OMX_BF16, w.codes, w.scales, 32, OMX_I8_BLOCKED, nullptr, lr, y_f32,
@@ -172,7 +191,7 @@ int32_t forward(olora* t) {
   TRY(omx_rms_norm_forward(ctx, t->layers[0].x, OMX_F32, t->norm(0, 0), t->layers[0].h1, OMX_BF16, N, d, eps));
   for (uint32_t l = 0; l < c.layers; ++l) {
     olora::Layer& A = t->layers[l];
-    for (QMat* w : {&A.qkv, &A.o, &A.gu, &A.dn}) w->formed = 0;
+    TRY(copies_of_layer(t, A));
     const bool last = l + 1 == c.layers;
     // h A^T for the three sites at once: [N, 3r] in the first columns of ha.
     TRY(omx_gemm_pitched(ctx, A.h1, d, 1, t->a16(l, 0), 1, d, OMX_BF16, A.ha, OMX_BF16, 4 * r, N, d, 3 * r, 0));

@@ -528,10 +528,17 @@ def test_a_kept_copy_of_a_weight_gives_the_bits_of_a_copy_of_its_own(rows, kin, 
             tails = [tuple(be.upload(r.normal(0, 0.1, (n, rank)).astype(np.float32), BF16) for n in (rows, cols)) + (0,) for cols in (nout, kin)]
 
         def both(copies, formed=None):
-            ys, left = [], []
+            ys, left, first = [], [], [0, 0]
+            if copies == "in one launch":
+                marks, many = (C.c_uint64 * 2)(), lambda xs: (C.c_uint64 * 2)(*xs)
+                be._check(be._lib.omx_i8_copies_form(
+                    be._ctx, (C.c_void_p * 2)(*(w[0].ptr for w in ws)), (C.c_void_p * 2)(*(w[1].ptr for w in ws)), many([nout] * 2), many([kin] * 2),
+                    many([0, size]), C.c_uint64(2), C.c_uint64(2 * size), C.c_uint64(32), C.c_int32(0), C.c_uint64(rows), marks))
+                first = list(marks)
+                assert all(first)
             for i, w in enumerate(ws):
                 if copies:
-                    be._check(be._lib.omx_i8_copy_next(be._ctx, C.c_uint64(i * size), C.c_uint64(2 * size), C.c_uint64(0)))
+                    be._check(be._lib.omx_i8_copy_next(be._ctx, C.c_uint64(i * size), C.c_uint64(2 * size), C.c_uint64(first[i])))
                 ys.append(be.linear_i8_group_forward(x, *w, low_rank=tails[0]))
                 left.append(formed or be._lib.omx_i8_copy_formed(be._ctx))
             yield left
@@ -547,6 +554,7 @@ def test_a_kept_copy_of_a_weight_gives_the_bits_of_a_copy_of_its_own(rows, kin, 
         left, got = both(True)
         assert left[0] != 0 and left[0] == left[1]
         assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        assert all(np.array_equal(a, b) for a, b in zip(list(both("in one launch"))[1], want))
         _, got = both(True, formed=left[0] + 7)  # not this block's: formed anew
         assert all(np.array_equal(a, b) for a, b in zip(got, want))
         pair = both(True)
