@@ -32,8 +32,8 @@ struct GemmArgs {
   // Strided batch: block (x, y) works on product y, whose operands start batch_* BYTES after
   // product y - 1's. batches == 1 for a single product.
   int batches;
-  long batch_a, batch_b, batch_c;
   int symmetric;  // C (bf16, square) equals its transpose: tiles below the diagonal are not formed but stored with those above
+  long batch_a, batch_b, batch_c;
 };
 
 // Tiles of a symmetric output of `m` rows that are formed: those not wholly below the diagonal.
