@@ -1163,7 +1163,9 @@ __device__ __forceinline__ void key_sample_sum(const unsigned short* __restrict_
 // the cut tile cost registers this kernel does not have: with them it spills, and runs 11 % slower).
 // dS / scale = P (dP - delta) goes into dQ^T through the matrix units, and `ds_sum` collects this
 // lane's share of the row sum of its bf16 copy.
-template <int D, bool GENERAL>
+// IN_TURN as in the forward. At head_dim 64 with one group, in turn / left to the compiler: 8 x 12 x 1024 42.2 / 41.2 us, 16 x 12 x 1024
+// 66.9 / 65.8, 8 x 12 x 640 22.0 / 21.6, but 12 x 12 over 3 x 999 53.2 / 55.3: left.
+template <int D, bool GENERAL, bool IN_TURN>
 __device__ __forceinline__ void flash_dq_tile(const char* k_rows, const char* v_rows, const u32x4 (&qf)[D / 16],
                                               const u32x4 (&gf)[D / 16], floatx16 (&dq)[D / 32], float& ds_sum,
                                               float scale_log2, float neg_lse, float row_del, int key0, int q_row, int T,
@@ -1173,11 +1175,19 @@ __device__ __forceinline__ void flash_dq_tile(const char* k_rows, const char* v_
 #pragma unroll
   for (int sub = 0; sub < 2; ++sub) {
     floatx16 sc = zero16(), dp = zero16();
-    in_turn<2 * KK>([&](auto i) { return frag_rows<D>(i.value % 2 ? v_rows : k_rows, sub, i.value / 2, l32, lg); },
-                                    [&](auto i, const u32x4& f) {
-                                      if constexpr (i.value % 2 == 0) sc = mfma(f, qf[i.value / 2], sc);
-                                      else dp = mfma(f, gf[i.value / 2], dp);
-                                    });
+    if constexpr (IN_TURN) {
+      in_turn<2 * KK>([&](auto i) { return frag_rows<D>(i.value % 2 ? v_rows : k_rows, sub, i.value / 2, l32, lg); },
+                      [&](auto i, const u32x4& f) {
+                        if constexpr (i.value % 2 == 0) sc = mfma(f, qf[i.value / 2], sc);
+                        else dp = mfma(f, gf[i.value / 2], dp);
+                      });
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        sc = mfma(frag_rows<D>(k_rows, sub, kk, l32, lg), qf[kk], sc);
+        dp = mfma(frag_rows<D>(v_rows, sub, kk, l32, lg), gf[kk], dp);
+      }
+    }
     if constexpr (GENERAL) {
 #pragma unroll
       for (int vv = 0; vv < 16; ++vv) {
@@ -1191,15 +1201,25 @@ __device__ __forceinline__ void flash_dq_tile(const char* k_rows, const char* v_
       const float p = __builtin_amdgcn_exp2f(fmaf(sc[vv], scale_log2, neg_lse));
       dp[vv] = p * (dp[vv] - row_del);  // dS / scale: the scale joins dQ at the end
     }
-    u32x4 dsb;
-    in_turn<2 * MT>([&](auto i) { return frag_tr<D>(k_rows, i.value % MT, sub, i.value / MT, lane); },
-                                    [&](auto i, const u32x4& f) {
-                                      if constexpr (i.value % MT == 0) {
-                                        dsb = pack8(dp, i.value / MT);
-                                        ds_sum = sum_pairs(dsb.x, sum_pairs(dsb.y, sum_pairs(dsb.z, sum_pairs(dsb.w, ds_sum))));
-                                      }
-                                      dq[i.value % MT] = mfma(f, dsb, dq[i.value % MT]);
-                                    });
+    if constexpr (IN_TURN) {
+      u32x4 dsb;
+      in_turn<2 * MT>([&](auto i) { return frag_tr<D>(k_rows, i.value % MT, sub, i.value / MT, lane); },
+                      [&](auto i, const u32x4& f) {
+                        if constexpr (i.value % MT == 0) {
+                          dsb = pack8(dp, i.value / MT);
+                          ds_sum = sum_pairs(dsb.x, sum_pairs(dsb.y, sum_pairs(dsb.z, sum_pairs(dsb.w, ds_sum))));
+                        }
+                        dq[i.value % MT] = mfma(f, dsb, dq[i.value % MT]);
+                      });
+    } else {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const u32x4 dsb = pack8(dp, c);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) dq[mt] = mfma(frag_tr<D>(k_rows, mt, sub, c, lane), dsb, dq[mt]);
+        ds_sum = sum_pairs(dsb.x, sum_pairs(dsb.y, sum_pairs(dsb.z, sum_pairs(dsb.w, ds_sum))));
+      }
+    }
   }
 }
 
@@ -1310,18 +1330,18 @@ __device__ __forceinline__ void flash_dq_blocks(
         advance(kt);
         const int key0 = kt * 64;
         if ((GROUPS == 1 || kt <= kt_last) && key0 <= wave_q0 + 31 && key0 + 63 + s.window > wave_q0)
-          flash_dq_tile<D, true>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, key0, q_row, T, s.window,
+          flash_dq_tile<D, true, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, key0, q_row, T, s.window,
                                  lane);
       }
     } else if (wave_q0 < T) {
       const int diag_kt = wave_q0 / 64;
       for (; kt < diag_kt; kt += GROUPS) {
         advance(kt);
-        flash_dq_tile<D, false>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, kt * 64, q_row, T, 0, lane);
+        flash_dq_tile<D, false, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, kt * 64, q_row, T, 0, lane);
       }
       if (GROUPS == 1 || kt == diag_kt) {
         advance(kt);
-        flash_dq_tile<D, true>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, kt * 64, q_row, T, 0, lane);
+        flash_dq_tile<D, true, flash_in_turn(D, GROUPS)>(k_rows, v_rows, qf, gf, dq, ds_sum, scale_log2, neg_lse, row_del, kt * 64, q_row, T, 0, lane);
         kt += GROUPS;
       }
     }
