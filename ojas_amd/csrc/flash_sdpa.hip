@@ -1612,6 +1612,9 @@ FlashKeyPlan flash_key_plan(omx_ctx* ctx, const FlashShape& s, int dim) {
 // takes 0.7 % more than the best of all, 22 % less than two launches. Left to two: many workgroups, where the dQ pass alone has three
 // per compute unit (16 x 16 x 256: 32.6 / 36.3; head_dim 128, 13 x 12 x 256: 53 / 54, x 512 101 / 131), and many query heads over a KV
 // head, whose tiles one workgroup walks (6 x 12 over 3 x 256: 29.1 / 29.7; the parts of flash_key_plan take those).
+// Under a window of at most 129 keys no workgroup walks far, however long the sequence, and one launch stays ahead with more of them: 8 x 12
+// heads, window 100, x 640 41 / 36; window 64, x 1000 49 / 46; 16 x 16, window 128, x 260 44 / 42; head_dim 128, 8 x 12, window 100, x 256
+// 42 / 36; x 320 (2.25 blocks a unit) 44 / 44.
 // Gradients over what the other pass still reads take two launches too, as they always could.
 int flash_together(omx_ctx* ctx, const FlashShape& s, int dim, const void* q, const void* k, const void* v, const void* out, const void* resid,
                    const void* gy, const void* gq, const void* gk, const void* gv) {
@@ -1624,7 +1627,8 @@ int flash_together(omx_ctx* ctx, const FlashShape& s, int dim, const void* q, co
     const long ones = (s.time + 127) / 128 * planes, fours = (s.time + 31) / 32 * planes;
     const bool few = dim == 64 ? (tiles <= 13 && 8 * ones <= 25 * units && (s.rep == 1 || s.rep * tiles <= 16)) || (s.rep == 1 && fours <= units)
                                : (ones <= units || (tiles >= 5 && 8 * ones <= 15 * units)) && (s.rep == 1 || s.rep * tiles <= 12);
-    if (!few) return 0;
+    const bool narrow = s.window > 0 && tiles <= 4 && s.rep == 1 && 2 * ones <= (dim == 64 ? 12 : 3) * units;
+    if (!few && !narrow) return 0;
   }
   struct Range {
     const char *first, *end;

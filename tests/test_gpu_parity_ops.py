@@ -558,7 +558,7 @@ def test_f32_attention_backward_in_one_launch_has_the_bits_of_two(be, shape, hkv
 @pytest.mark.parametrize("schedule", [1, 3, 4])
 @pytest.mark.parametrize("shape,hkv,window", [((1, 1, 1, 64), 1, None), ((2, 2, 63, 64), 2, None), ((1, 4, 65, 128), 2, None), ((2, 8, 128, 64), 2, 33),
                                               ((3, 5, 129, 64), 5, None), ((1, 2, 200, 128), 2, 50), ((2, 3, 333, 64), 3, 64), ((1, 1, 1024, 64), 1, None),
-                                              ((1, 1, 1000, 128), 1, 300), ((1, 16, 64, 64), 1, None)])
+                                              ((1, 1, 1000, 128), 1, 300), ((1, 16, 64, 64), 1, None), ((8, 12, 400, 64), 12, 100)])
 def test_bf16_attention_backward_in_one_launch_has_the_bits_of_two(be, shape, hkv, window, schedule):
     """Both passes of the bf16 backward in one launch on one, two and four groups of waves, the key side's row terms formed there: every
     bit of two launches, last tiles and row blocks past the end, groups of heads and windows among them. Gradients in place of
